@@ -126,6 +126,21 @@ int mg_neighbour_cell_order(const void* workspace, size_t workspace_bytes, int b
                             float cutoff, float box_x, float box_y, float box_z,
                             int* order /* batch*nodes */, mg_stream_t stream);
 
+/* The whole radius graph as the models use it (Graph.radius_graph and the edge vectors of graph_setup,
+ * managan/graph_layers.py:25-34,62-66, archs/meanflow_painn8.py:167-172) in as few launches as possible: two for a graph of at
+ * most 16384 atoms in boxes of at most 2048, five for eight boxes of 16384.  mg_graph_search bins, sorts and counts into
+ * the workspace; mg_graph_fill then writes row_ptr, edge_counts and stats as mg_neighbour_count does (stats[3] also has
+ * bit 2, value 4, set when a coordinate is NaN), and per edge src and dst, optionally (non-null) their int64 copies and
+ * r_ij = boxwrap(box, x[dst] - x[src]), optionally the cell order of the atoms.  Edges at positions from `capacity` on
+ * are dropped while row_ptr stays exact: a caller whose estimate was too small repeats mg_graph_fill with larger arrays. */
+int mg_graph_search(const float* x /* (batch,nodes,3) */, int batch, int nodes, float cutoff, float box_x, float box_y,
+                    float box_z, void* workspace, size_t workspace_bytes, mg_stream_t stream);
+int mg_graph_fill(const float* x, const void* workspace, size_t workspace_bytes, int batch, int nodes, float cutoff,
+                  float box_x, float box_y, float box_z, int* row_ptr /* batch*nodes+1 */, int* edge_counts /* batch */,
+                  int* stats /* 4 */, int capacity, int* src /* capacity */, int* dst /* capacity */,
+                  int64_t* src64 /* capacity or null */, int64_t* dst64, float* r_ij /* (capacity,3) or null */,
+                  int* order /* batch*nodes or null */, mg_stream_t stream);
+
 /* First step of the search on its own: wrapped positions (batch,nodes,3) and box-local
  * linear cell ids (batch,nodes), as assignParticlesToCells computes them
  * (extensions/neighbour_grid/neighbour_grid_kern.cu:75-82).  Diagnostic / test entry. */

@@ -13,10 +13,12 @@
 //            64 at a time, counting hits with ballot/popcount -> degree; the hits
 //            themselves go, in window order, into the atom's row of a scratch
 //            array (hit rows of a fixed capacity)
+//            (boxes of at most 2048 atoms and 4096 cells: bin, sort and count are one kernel, box_search_kernel)
 //   scan     degrees -> CSR row_ptr (+ per-box edge counts, statistics)
 //   fill     copies the hit rows to row_ptr[i] (exact-size rows, no atomics per
 //            edge, no geometry); a row with more hits than a hit row holds is
-//            swept again by one wave
+//            swept again by one wave.  graph_fill_kernel (mg_graph_fill) is scan and fill in one, and writes int64
+//            indices, edge vectors and the cell order as well
 //
 // fp32 recipe (this file is compiled with -ffp-contract=off):
 //   w    = remainderf(x - box/2, box) + box/2                 (IEEE remainder)
@@ -73,6 +75,9 @@ struct Grid {
     int batch, nodes;
 };
 
+constexpr int kNanBit = 1 << 30;    // in box_max; a cell holds fewer than 2^30 atoms
+constexpr int kNanCell = 1 << 31;   // in cell_of: the atom has a NaN coordinate (consumers mask it out)
+
 struct Workspace {
     float4* wrapped;    // A: (w.x, w.y, w.z, bits of box-local index)
     float4* sorted;     // A: same records in cell order
@@ -86,7 +91,8 @@ struct Workspace {
     int* block_max;     // scan scratch
     int* deg_sums;      // sums / maxima of the degrees per tile of kScanTile rows
     int* deg_max;
-    int* box_max;       // batch: largest cell occupancy of each box (per-box sort)
+    int* box_max;       // largest cell occupancy per workgroup of the sort, bit kNanBit: the box holds a NaN coordinate
+                        // (without the per-box sort: one occupancy, one flag)
     void* hits;         // A x hit_cap: neighbours found by the count pass (box-local atom ids, window order);
                         // 16-bit entries when a box has at most 65536 atoms, else 32-bit
     int hit_cap;        // entries per hit row; rows with more hits are recomputed by the fill pass
@@ -117,7 +123,7 @@ Workspace carve(void* base, long A, long C, int hit_cap, int hit_bytes) {
     w.block_max = static_cast<int*>(take(sizeof(int) * scan_blocks));
     w.deg_sums = static_cast<int*>(take(sizeof(int) * scan_blocks));
     w.deg_max = static_cast<int*>(take(sizeof(int) * scan_blocks));
-    w.box_max = static_cast<int*>(take(sizeof(int) * (A > 0 ? A : 1)));   // (batch <= A)
+    w.box_max = static_cast<int*>(take(sizeof(int) * (A + 2)));           // (batch <= A)
     w.hits = take((size_t)hit_bytes * A * hit_cap);
     w.hit_cap = hit_cap;
     w.hit_bytes = hit_bytes;
@@ -145,17 +151,63 @@ int make_grid(float cutoff, float bx, float by, float bz, int batch, int nodes, 
 }
 
 // ---------------------------------------------------------------- device math
+// The IEEE remainder is exact, so t - n box in one fma is the remainder bit for bit whenever n is its multiple, and a
+// multiple that is off by one or more leaves at least box / 2: only results near box / 2 (and non-finite input) need
+// the library's loop.
 __device__ __forceinline__ float wrap_into_box(float x, float box) {
     const float half = 0.5f * box;
-    return remainderf(x - half, box) + half;
+    const float t = x - half;
+    const float r = __fmaf_rn(-rintf(t * (1.0f / box)), box, t);
+    if (fabsf(r) < 0.4999f * box) return r + half;
+    return remainderf(t, box) + half;
 }
 
+// (int)(correctly rounded quotient) % ndiv.  The quotient with a reciprocal is within a few ulp of the correctly
+// rounded one: where both ends of that interval truncate to the same integer, so does the quotient.
 __device__ __forceinline__ int cell_coord(float w, float box, int ndiv) {
     const float scaled = (float)ndiv * w;
-    const float q = __fdiv_rn(scaled, box);
-    int c = ((int)q) % ndiv;
+    const float q = scaled * (1.0f / box);
+    int c = (int)(q * 0.9999995f);
+    if (!(c == (int)(q * 1.0000005f) && q >= 0.f)) c = (int)__fdiv_rn(scaled, box);
+    if (c >= ndiv) c %= ndiv;
     return c < 0 ? 0 : c;   // only reachable with non-finite input
 }
+
+// torch's float `%` (floor-mod, b > 0): fmod, then move a result of the wrong sign by one period
+__device__ __forceinline__ float floor_mod(float a, float b) {
+    float m = fmodf(a, b);
+    if (m < 0.f) m += b;
+    return m;
+}
+
+// boxwrap(box, x_j - x_i), a floor-mod per axis.  fmod is exact, so one fma gives it bit for bit whenever the quotient
+// was truncated to the right integer, which the result's range shows; fmodf itself (a loop over the exponents'
+// difference) is left for the rest, behind one branch for the three axes.
+struct Box3 {
+    float x, y, z, ix, iy, iz;
+};
+__device__ __forceinline__ bool fast_wrap(float raw, float box, float inv_box, float* r) {
+    const float half = 0.5f * box, a = raw + half;
+    const float m = __fmaf_rn(-truncf(a * inv_box), box, a);
+    *r = (m < 0.f ? m + box : m) - half;
+    return fabsf(m) < box && (a < 0.f ? m <= 0.f : m >= 0.f);
+}
+__device__ __forceinline__ float3 wrapped_difference(const float3& xj, const float3& xi, const Box3& box) {
+    const float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
+    float3 r;
+    const bool fast_x = fast_wrap(dx, box.x, box.ix, &r.x), fast_y = fast_wrap(dy, box.y, box.iy, &r.y);
+    const bool fast_z = fast_wrap(dz, box.z, box.iz, &r.z);
+    if (!(fast_x && fast_y && fast_z)) {
+        r.x = floor_mod(dx + 0.5f * box.x, box.x) - 0.5f * box.x;
+        r.y = floor_mod(dy + 0.5f * box.y, box.y) - 0.5f * box.y;
+        r.z = floor_mod(dz + 0.5f * box.z, box.z) - 0.5f * box.z;
+    }
+    return r;
+}
+__device__ __forceinline__ Box3 box_of(float bx, float by, float bz) {
+    return Box3{bx, by, bz, 1.0f / bx, 1.0f / by, 1.0f / bz};
+}
+__device__ __forceinline__ float3 load3(const float* p) { return make_float3(p[0], p[1], p[2]); }
 
 __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
 #pragma unroll
@@ -186,16 +238,19 @@ __global__ void __launch_bounds__(256) bin_kernel(const float* __restrict__ x, G
     if (a >= A) return;
     const int b = (int)(a / g.nodes);
     const int i = (int)(a - (long)b * g.nodes);
-    const float wx = wrap_into_box(x[3 * a + 0], g.bx);
-    const float wy = wrap_into_box(x[3 * a + 1], g.by);
-    const float wz = wrap_into_box(x[3 * a + 2], g.bz);
+    const float px = x[3 * a + 0], py = x[3 * a + 1], pz = x[3 * a + 2];
+    const float wx = wrap_into_box(px, g.bx), wy = wrap_into_box(py, g.by), wz = wrap_into_box(pz, g.bz);
     const int cx = cell_coord(wx, g.bx, g.nx);
     const int cy = cell_coord(wy, g.by, g.ny);
     const int cz = cell_coord(wz, g.bz, g.nz);
     const int cell = ((b * g.nx + cx) * g.ny + cy) * g.nz + cz;
+    const bool nan = px != px || py != py || pz != pz;
     w.wrapped[a] = make_float4(wx, wy, wz, __int_as_float(i));
-    w.cell_of[a] = cell;
-    if (HIST) w.slot[a] = atomicAdd(&w.cell_count[cell], 1);
+    w.cell_of[a] = cell | (nan && !HIST ? kNanCell : 0);
+    if (HIST) {
+        w.slot[a] = atomicAdd(&w.cell_count[cell], 1);
+        if (nan) atomicOr(&w.box_max[1], kNanBit);
+    }
 }
 
 // Counting sort of a box by cell, entirely in LDS: histogram (LDS atomics), scan, placement, rank by atom id inside
@@ -214,6 +269,7 @@ __global__ void __launch_bounds__(kSortThreads) sort_box_kernel(Grid g, Workspac
     // rank loop may read past the end of its cell without a bounds check (the array ends in 8 keys of INT_MAX)
     __shared__ int placed[kSortNodes + 8 + 1];   // (+ a spare word that takes the writes for atoms of other slabs)
     __shared__ int wave_sum[kSortThreads / kWave], wave_max[kSortThreads / kWave], wave_before[kSortThreads / kWave];
+    __shared__ int wave_nan[kSortThreads / kWave];
     const int slab = blockIdx.x, slabs = gridDim.x;
     const int b = blockIdx.y, tid = threadIdx.x;
     const int lane = tid & (kWave - 1), wave = tid / kWave;
@@ -224,7 +280,7 @@ __global__ void __launch_bounds__(kSortThreads) sort_box_kernel(Grid g, Workspac
     for (int c = tid; c <= ncs + kWave; c += kSortThreads) start[c] = 0;
     __syncthreads();
     int cl[kPer], sl[kPer];                   // cell within the slab (-1: another slab's atom), slot within the cell
-    int n_before = 0;
+    int n_before = 0, nan = 0;
     // Straight-line code, so that the 16 loads (and then the 16 LDS atomics) of a thread are in flight together:
     // an index past the box reads the box's last atom and is discarded, an atom of another slab counts into a
     // spare bin of its lane.
@@ -233,8 +289,9 @@ __global__ void __launch_bounds__(kSortThreads) sort_box_kernel(Grid g, Workspac
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
         const int i = tid + kSortThreads * j;
-        const int c = cells[i < g.nodes ? i : last] - cell_base;
-        cl[j] = i < g.nodes ? c : g.ncells;
+        const int c = cells[i < g.nodes ? i : last];
+        nan |= c;                             // (the sign bit)
+        cl[j] = i < g.nodes ? (c & ~kNanCell) - cell_base : g.ncells;
     }
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
@@ -246,6 +303,8 @@ __global__ void __launch_bounds__(kSortThreads) sort_box_kernel(Grid g, Workspac
     }
     for (int d = kWave / 2; d > 0; d >>= 1) n_before += __shfl_xor(n_before, d);
     if (lane == 0) wave_before[wave] = n_before;
+    const int any_nan = __any(nan < 0);
+    if (lane == 0) wave_nan[wave] = any_nan;
     __syncthreads();
     // exclusive scan of the cell sizes: a thread owns kCellsPer consecutive cells
     int cnt[kCellsPer], sum = 0, mx = 0;
@@ -278,9 +337,9 @@ __global__ void __launch_bounds__(kSortThreads) sort_box_kernel(Grid g, Workspac
     }
     if (tid == 0) {
         start[ncs] = mine;
-        int m = 0;
-        for (int k = 0; k < kSortThreads / kWave; k++) m = wave_max[k] > m ? wave_max[k] : m;
-        w.box_max[b * slabs + slab] = m;
+        int m = 0, any = 0;
+        for (int k = 0; k < kSortThreads / kWave; k++) { m = wave_max[k] > m ? wave_max[k] : m; any |= wave_nan[k]; }
+        w.box_max[b * slabs + slab] = m | (any ? kNanBit : 0);
         if (b == g.batch - 1 && slab == slabs - 1) w.cell_start[(long)g.batch * g.ncells] = g.batch * g.nodes;
     }
     __syncthreads();
@@ -456,7 +515,7 @@ __global__ void __launch_bounds__(kScanThreads) scan_apply_kernel(const int* __r
     if (totals && box_max != nullptr && threadIdx.x < kWave) {
         // largest cell occupancy over the boxes (the per-box sort leaves one value per box)
         int m = 0;
-        for (int k = threadIdx.x; k < n_box; k += kWave) m = box_max[k] > m ? box_max[k] : m;
+        for (int k = threadIdx.x; k < n_box; k += kWave) { const int v = box_max[k] & ~kNanBit; m = v > m ? v : m; }
         for (int d = kWave / 2; d > 0; d >>= 1) { const int t = __shfl_xor(m, d); m = t > m ? t : m; }
         if (threadIdx.x == 0) *out_box_max = m;
     }
@@ -675,16 +734,41 @@ __global__ void __launch_bounds__(256) count_kernel(Grid g, Workspace w) {
     }
 }
 
+// What the fill pass writes per edge: the int32 indices, and for a caller that asked for them their int64 copies and
+// the edge vector boxwrap(box, x_j - x_i).
+struct EdgeOut {
+    int* src;
+    int* dst;
+    int64_t* src64;     // both or neither
+    int64_t* dst64;
+    float* r_ij;        // or null
+    const float* x;     // unwrapped positions (with r_ij)
+
+    __device__ __forceinline__ void store(int e, int i, int j) const {
+        src[e] = i;
+        dst[e] = j;
+        if (src64) {
+            src64[e] = i;
+            dst64[e] = j;
+        }
+    }
+    __device__ __forceinline__ void store_vector(int e, const float3& r) const {
+        float* to = r_ij + 3 * (long)e;
+        to[0] = r.x;
+        to[1] = r.y;
+        to[2] = r.z;
+    }
+};
+
 // Fill pass, slow path: one wave sweeps the window of atom `row` again (candidates from global memory, all axes with
 // the minimum image) and writes its hits at out_pos, in window order.  For rows whose hit row was too short.
-__device__ void refill_row(const Grid& g, const Workspace& w, int row, int out_pos, int capacity,
-                           int* __restrict__ src, int* __restrict__ dst) {
+__device__ void refill_row(const Grid& g, const Workspace& w, int row, int out_pos, int capacity, const EdgeOut& out) {
     const int lane = threadIdx.x & (kWave - 1);
     const int b = row / g.nodes;
     const int id_self = row - b * g.nodes;
     const int node_base = b * g.nodes;
     const float4 self = w.wrapped[row];
-    int c = w.cell_of[row] - b * g.ncells;
+    int c = (w.cell_of[row] & ~kNanCell) - b * g.ncells;
     const int cz = c % g.nz;
     c /= g.nz;
     const int cy = c % g.ny, cx = c / g.ny;
@@ -722,8 +806,10 @@ __device__ void refill_row(const Grid& g, const Workspace& w, int row, int out_p
         const unsigned long long mask = __ballot(hit);
         const int pos = out_pos + hits_below(mask, cnt);
         if (hit && pos >= 0 && pos < capacity) {
-            src[pos] = row;
-            dst[pos] = node_base + other;
+            out.store(pos, row, node_base + other);
+            if (out.r_ij)
+                out.store_vector(pos, wrapped_difference(load3(out.x + 3 * (long)(node_base + other)), load3(out.x + 3 * (long)row),
+                                                         box_of(g.bx, g.by, g.bz)));
         }
         cnt += __popcll(mask);
     }
@@ -735,7 +821,7 @@ __device__ void refill_row(const Grid& g, const Workspace& w, int row, int out_p
 constexpr int kFillRows = 64;
 template <typename HitT>
 __global__ void __launch_bounds__(256) fill_kernel(Grid g, Workspace w, const int* __restrict__ row_ptr,
-                                                   int* __restrict__ src, int* __restrict__ dst, int capacity) {
+                                                   EdgeOut out, int capacity) {
     __shared__ int rp[kFillRows + 1];
     __shared__ int first_row[kFillRows];      // first row of the box that the row belongs to
     const long A = (long)g.batch * g.nodes;
@@ -755,15 +841,318 @@ __global__ void __launch_bounds__(256) fill_kernel(Grid g, Workspace w, const in
             if (rp[mid] <= e) lo = mid; else hi = mid - 1;
         }
         const int idx = e - rp[lo], deg = rp[lo + 1] - rp[lo];
-        if (deg <= cap && idx >= 0 && idx < deg && e >= 0 && e < capacity) {
-            src[e] = (int)(r0 + lo);
-            dst[e] = first_row[lo] + (int)hits[(r0 + lo) * cap + idx];
-        }
+        if (deg <= cap && idx >= 0 && idx < deg && e >= 0 && e < capacity)
+            out.store(e, (int)(r0 + lo), first_row[lo] + (int)hits[(r0 + lo) * cap + idx]);
     }
     // rows with more hits than a hit row holds: a wave each
     const int wave = threadIdx.x / kWave;
     for (int r = wave; r < nrows; r += 256 / kWave)
-        if (rp[r + 1] - rp[r] > cap) refill_row(g, w, (int)(r0 + r), rp[r], capacity, src, dst);
+        if (rp[r + 1] - rp[r] > cap) refill_row(g, w, (int)(r0 + r), rp[r], capacity, out);
+}
+
+// Small boxes: binning, sort and count in ONE kernel.  gridDim.x workgroups share a box; each bins and sorts the whole
+// box in LDS (a few thousand clocks for at most kBoxNodes atoms: cheaper than the two launches and the round trip through
+// memory it replaces) and then counts the home cells blockIdx.x * 8 + wave, + 8 gridDim.x, ...: a wave takes a home
+// cell, its lanes hold one group of 64 candidates of the window at a time in registers, and every home atom of the cell
+// sweeps them; lane h keeps the running count of home atom h.  Same hit rows, degrees and tables as the separate kernels.
+// What bounds it is latency (a dozen dependent LDS phases); 2 launches per search instead of 6 + (see graph_fill_kernel).
+constexpr int kBoxThreads = 512, kBoxNodes = 2048, kBoxCells = 4096, kBoxWaves = kBoxThreads / kWave;
+template <int kPer, typename HitT>
+__global__ void __launch_bounds__(kBoxThreads) box_search_kernel(const float* __restrict__ x, Grid g, Workspace w) {
+    constexpr int kNodes = kPer * kBoxThreads;
+    __shared__ float4 sorted[kNodes];
+    __shared__ int placed[kNodes + 8];            // keys (cell << 11 | atom): see sort_box_kernel
+    __shared__ int start[kBoxCells + 1];
+    __shared__ int wave_sum[kBoxWaves], wave_max[kBoxWaves], wave_nan[kBoxWaves];
+    const int part = blockIdx.x, parts = gridDim.x, b = blockIdx.y, tid = threadIdx.x;
+    const int lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const long base = (long)b * g.nodes;
+    const int cell_base = b * g.ncells;
+
+    float4 rec[kPer];
+    int cl[kPer], sl[kPer], nan = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; j++) {
+        const int i = tid + kBoxThreads * j;
+        cl[j] = -1;
+        if (i < g.nodes) {
+            const float* p = x + 3 * (base + i);
+            const float px = p[0], py = p[1], pz = p[2];
+            nan |= (px != px || py != py || pz != pz) ? 1 : 0;
+            rec[j] = make_float4(wrap_into_box(px, g.bx), wrap_into_box(py, g.by), wrap_into_box(pz, g.bz), __int_as_float(i));
+            cl[j] = (cell_coord(rec[j].x, g.bx, g.nx) * g.ny + cell_coord(rec[j].y, g.by, g.ny)) * g.nz +
+                    cell_coord(rec[j].z, g.bz, g.nz);
+        }
+    }
+    for (int c = tid; c <= g.ncells; c += kBoxThreads) start[c] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kPer; j++)
+        if (cl[j] >= 0) sl[j] = atomicAdd(&start[cl[j]], 1);
+    __syncthreads();
+    // exclusive scan of the cell sizes: a thread owns `per` consecutive cells
+    const int per = (g.ncells + kBoxThreads - 1) / kBoxThreads;
+    int sum = 0, mx = 0;
+    for (int k = 0; k < per; k++) {
+        const int c = tid * per + k;
+        const int v = c < g.ncells ? start[c] : 0;
+        sum += v;
+        mx = v > mx ? v : mx;
+    }
+    const int incl = wave_incl_scan(sum, lane);
+    for (int d = kWave / 2; d > 0; d >>= 1) { const int t = __shfl_xor(mx, d); mx = t > mx ? t : mx; }
+    const int any_nan = __any(nan);
+    if (lane == kWave - 1) wave_sum[wave] = incl;
+    if (lane == 0) { wave_max[wave] = mx; wave_nan[wave] = any_nan; }
+    __syncthreads();
+    int run = incl - sum;
+    for (int k = 0; k < wave; k++) run += wave_sum[k];
+    for (int k = 0; k < per; k++) {
+        const int c = tid * per + k;
+        if (c < g.ncells) {
+            const int v = start[c];
+            start[c] = run;
+            run += v;
+        }
+    }
+    if (tid == 0) start[g.ncells] = g.nodes;
+    if (tid < 8) placed[g.nodes + tid] = 0x7fffffff;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kPer; j++)
+        if (cl[j] >= 0) placed[start[cl[j]] + sl[j]] = (cl[j] << 11) | (tid + kBoxThreads * j);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kPer; j++) {
+        if (cl[j] < 0) continue;
+        const int key = (cl[j] << 11) | (tid + kBoxThreads * j);
+        const int lo = start[cl[j]], hi = start[cl[j] + 1];
+        int rank = 0;
+        for (int q0 = lo; q0 < hi; q0 += 8) {
+            int v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = placed[q0 + u];      // (q0 < nodes: at most 7 entries into the sentinels)
+#pragma unroll
+            for (int u = 0; u < 8; u++) rank += v[u] < key ? 1 : 0;
+        }
+        sorted[lo + rank] = rec[j];
+        if (part == 0) {                          // (the fill pass sweeps rows that overflow their hit row again)
+            w.wrapped[base + tid + kBoxThreads * j] = rec[j];
+            w.cell_of[base + tid + kBoxThreads * j] = cell_base + cl[j];
+        }
+    }
+    if (part == 0) {
+        for (int c = tid; c < g.ncells; c += kBoxThreads) w.cell_start[cell_base + c] = (int)base + start[c];
+        if (tid == 0) {
+            int m = 0, any = 0;
+            for (int k = 0; k < kBoxWaves; k++) { m = wave_max[k] > m ? wave_max[k] : m; any |= wave_nan[k]; }
+            w.box_max[b] = m | (any ? kNanBit : 0);
+            if (b == g.batch - 1) w.cell_start[(long)g.batch * g.ncells] = g.batch * g.nodes;
+        }
+    }
+    __syncthreads();
+    for (int p = tid + kBoxThreads * part; p < g.nodes; p += kBoxThreads * parts) w.sorted[base + p] = sorted[p];
+
+    const float ibx = 1.0f / g.bx, iby = 1.0f / g.by, ibz = 1.0f / g.bz;
+    HitT* const hits = static_cast<HitT*>(w.hits);
+    const int row_bytes = w.hit_cap * (int)sizeof(HitT);
+    for (int c = part * kBoxWaves + wave; c < g.ncells; c += parts * kBoxWaves) {        // uniform in the wave
+        const int home_lo = __builtin_amdgcn_readfirstlane(start[c]), home_hi = __builtin_amdgcn_readfirstlane(start[c + 1]);
+        if (home_lo == home_hi) continue;
+        const int cz = c % g.nz, cxy = c / g.nz, cy = cxy % g.ny, cx = cxy / g.ny;
+        const int t = lane < 27 ? lane : 26;
+        const int dx = t / 9 - 1, dy = (t / 3) % 3 - 1, dz = t % 3 - 1;
+        int nx = cx + dx, ny = cy + dy, nz = cz + dz;
+        nx = nx < 0 ? nx + g.nx : (nx >= g.nx ? nx - g.nx : nx);
+        ny = ny < 0 ? ny + g.ny : (ny >= g.ny ? ny - g.ny : ny);
+        nz = nz < 0 ? nz + g.nz : (nz >= g.nz ? nz - g.nz : nz);
+        const int nc = (nx * g.ny + ny) * g.nz + nz;
+        const int st = start[nc];
+        const int len = lane < 27 ? start[nc + 1] - st : 0;
+        int pre = len;
+#pragma unroll
+        for (int d = 1; d < 32; d <<= 1) {
+            const int up = __shfl_up(pre, d);
+            if (lane >= d) pre += up;
+        }
+        const int excl = pre - len;
+        const int M = __builtin_amdgcn_readlane(pre, 26);
+        const bool inner = g.nx >= 5 && cx >= 2 && cx <= g.nx - 3 && g.ny >= 5 && cy >= 2 && cy <= g.ny - 3 && g.nz >= 5 &&
+                           cz >= 2 && cz <= g.nz - 3;
+        for (int h0 = home_lo; h0 < home_hi; h0 += kWave) {          // (one trip unless a cell holds more than 64 atoms)
+            const int hn = home_hi - h0 < kWave ? home_hi - h0 : kWave;
+            int counts = 0;                                          // lane h: hits of home atom h0 + h so far
+            for (int k0 = 0; k0 < M; k0 += kWave) {
+                const int k = k0 + lane;
+                int lo = 0, hi = 26;                                 // last cell of the window with excl <= k
+#pragma unroll
+                for (int it = 0; it < 5; it++) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    const int pm = __shfl(excl, mid);
+                    if (pm <= k) lo = mid; else hi = mid - 1;
+                }
+                const int idx = __shfl(st, lo) + (k - __shfl(excl, lo));
+                const bool valid = k < M;
+                const float4 o = sorted[valid ? idx : home_lo];
+                for (int h = 0; h < hn; h++) {
+                    const float4 self = sorted[h0 + h];              // one address: a broadcast
+                    const bool close = inner ? within_cutoff<0>(self, o, g, ibx, iby, ibz)
+                                             : within_cutoff<7>(self, o, g, ibx, iby, ibz);
+                    const unsigned long long mask = __ballot(close && valid && idx != h0 + h);
+                    const int seen = __builtin_amdgcn_readlane(counts, h);
+                    const int row = (int)base + __builtin_amdgcn_readfirstlane(__float_as_int(self.w));
+                    const __amdgpu_buffer_rsrc_t hit_row =
+                        __builtin_amdgcn_make_buffer_rsrc(hits + (long)row * w.hit_cap, 0, row_bytes, 0x00020000);
+                    if (__builtin_amdgcn_inverse_ballot_w64(mask))
+                        store_hit(hit_row, __float_as_int(o.w), hits_below(mask, seen), HitT{});
+                    counts += lane == h ? __popcll(mask) : 0;
+                }
+            }
+            if (lane < hn) w.degree[base + __float_as_int(sorted[h0 + lane].w)] = counts;
+        }
+    }
+}
+
+// Row pointer, statistics and edges of a whole graph in one kernel.  A workgroup takes `rows_per` consecutive rows and
+// finds the position of its first edge by adding up the degrees of the rows before it: those of its tile of kScanTile
+// rows and the sums of the tiles before (tiled: scan_sums_kernel has left them), or simply all of them (at most
+// kDirectRows degrees from the L2: cheaper than a launch).  Workgroup 0 also reduces everything to the statistics.  The
+// edge's int64 indices and its vector are written here, where i and j are in registers, instead of by three kernels that
+// read the edge list back.  Bound by the stores, 36 bytes per edge with everything asked for, once a thread has several
+// edges' loads in flight: kFillUnroll edges at a time, rows found without branches.
+constexpr long kDirectRows = 16384;
+constexpr int kFillUnroll = 4;
+template <typename HitT>
+__global__ void __launch_bounds__(256) graph_fill_kernel(Grid g, Workspace w, int rows_per, int tiled, int n_box,
+                                                         int* __restrict__ row_ptr, int* __restrict__ edge_counts,
+                                                         int* stats, int capacity, EdgeOut out, int* __restrict__ order) {
+    __shared__ int rp[kFillRows + 1];
+    __shared__ int first_row[kFillRows];      // first row of the box that the row belongs to
+    __shared__ float3 x_row[kFillRows];
+    __shared__ long long wave_before[4], wave_all[4];
+    __shared__ int wave_mx[4], wave_cell[4], wave_flag[4];
+    const long A = (long)g.batch * g.nodes;
+    const long r0 = (long)blockIdx.x * rows_per;
+    const int nrows = A - r0 < rows_per ? (int)(A - r0) : rows_per;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    const bool totals = blockIdx.x == 0;
+    const int my_degree = (wave == 0 && lane < nrows) ? w.degree[r0 + lane] : 0;
+    const int tile = tiled ? (int)(r0 / kScanTile) : 0;
+    long long before = 0, all = 0;
+    int mx = 0, cell = 0, flag = 0;
+    if (tiled) {
+        for (int k = tid; k < tile; k += 256) before += w.deg_sums[k];
+        for (long r = (long)tile * kScanTile + tid; r < r0; r += 256) before += w.degree[r];
+    } else {
+        for (long r = tid; r < r0; r += 256) before += w.degree[r];
+    }
+    if (totals) {
+        const long n = tiled ? A / kScanTile + 1 : A;             // ceil((A + 1) / kScanTile) tiles
+        const int* sums = tiled ? w.deg_sums : w.degree;
+        const int* maxima = tiled ? w.deg_max : w.degree;
+        for (long k = tid; k < n; k += 256) {
+            all += sums[k];
+            const int m = maxima[k];
+            mx = m > mx ? m : mx;
+        }
+        for (int k = tid; k < n_box; k += 256) {
+            const int v = w.box_max[k] & ~kNanBit;
+            cell = v > cell ? v : cell;
+            flag |= w.box_max[k] & kNanBit;
+        }
+    }
+    for (int d = kWave / 2; d > 0; d >>= 1) {
+        before += __shfl_xor(before, d);
+        if (totals) {
+            all += __shfl_xor(all, d);
+            int t = __shfl_xor(mx, d);
+            mx = t > mx ? t : mx;
+            t = __shfl_xor(cell, d);
+            cell = t > cell ? t : cell;
+            flag |= __shfl_xor(flag, d);
+        }
+    }
+    if (lane == 0) {
+        wave_before[wave] = before;
+        wave_all[wave] = all;
+        wave_mx[wave] = mx;
+        wave_cell[wave] = cell;
+        wave_flag[wave] = flag;
+    }
+    __syncthreads();
+    if (totals && tid == 0) {
+        for (int k = 1; k < 4; k++) {
+            all += wave_all[k];
+            mx = wave_mx[k] > mx ? wave_mx[k] : mx;
+            cell = wave_cell[k] > cell ? wave_cell[k] : cell;
+            flag |= wave_flag[k];
+        }
+        // (a host may be polling these words: each is stored once, at system scope)
+        const int words[4] = {all > 0x7fffffffLL ? 0x7fffffff : (int)all, cell, mx,
+                              (all > 0x7fffffffLL ? 1 : 0) | (flag ? 4 : 0)};
+#pragma unroll
+        for (int k = 0; k < 4; k++) __hip_atomic_store(stats + k, words[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    if (wave == 0) {
+        const int first = (int)(wave_before[0] + wave_before[1] + wave_before[2] + wave_before[3]);
+        const int incl = wave_incl_scan(my_degree, lane);
+        if (lane < nrows) {
+            rp[lane + 1] = first + incl;
+            row_ptr[r0 + lane] = first + incl - my_degree;
+            const long next = r0 + lane + 1;
+            if (next == A) row_ptr[A] = first + incl;
+            const unsigned q = (unsigned)next / (unsigned)g.nodes;                // (next < 2^31: 32-bit divide)
+            if (q * (unsigned)g.nodes == (unsigned)next) edge_counts[q - 1] = first + incl;
+        }
+        if (lane == 0) rp[0] = first;
+    }
+    if (wave == 0 && lane >= nrows && lane < rows_per) rp[lane + 1] = 0x7fffffff;
+    if (wave == 1 && lane < nrows) {
+        const unsigned k = (unsigned)(r0 + lane);
+        const int first = (int)(k / (unsigned)g.nodes) * g.nodes;
+        first_row[lane] = first;
+        if (order) order[k] = first + __float_as_int(w.sorted[k].w);
+    }
+    if (wave == 2 && lane < nrows && out.r_ij) x_row[lane] = load3(out.x + 3 * (r0 + lane));
+    __syncthreads();
+    const int cap = w.hit_cap;
+    const HitT* __restrict__ hits = static_cast<const HitT*>(w.hits);
+    const int e_hi = rp[nrows];
+    const Box3 box = box_of(g.bx, g.by, g.bz);
+    for (int e0 = rp[0] + tid; e0 < e_hi; e0 += 256 * kFillUnroll) {
+        int row[kFillUnroll], j[kFillUnroll];
+        bool ok[kFillUnroll];
+#pragma unroll
+        for (int u = 0; u < kFillUnroll; u++) {
+            const int e = e0 + 256 * u;
+            int lo = 0;                                // last row with rp <= e (rp ends in INT_MAX past the last row)
+            for (int step = rows_per >> 1; step > 0; step >>= 1) lo += rp[lo + step] <= e ? step : 0;
+            lo = lo < nrows ? lo : nrows - 1;          // (a position past the last edge: discarded below, but it must not
+                                                       // name a row that is not staged, its atom is read all the same)
+            const int idx = e - rp[lo], deg = rp[lo + 1] - rp[lo];
+            ok[u] = e < e_hi && deg <= cap && idx >= 0 && idx < deg && e >= 0 && e < capacity;
+            row[u] = lo;
+            j[u] = ok[u] ? (int)hits[(r0 + lo) * cap + idx] : 0;
+        }
+        float3 xj[kFillUnroll];
+#pragma unroll
+        for (int u = 0; u < kFillUnroll; u++) {
+            j[u] += first_row[row[u]];
+            if (out.r_ij) xj[u] = load3(out.x + 3 * (long)j[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kFillUnroll; u++)
+            if (ok[u]) out.store(e0 + 256 * u, (int)r0 + row[u], j[u]);
+        if (out.r_ij) {
+#pragma unroll
+            for (int u = 0; u < kFillUnroll; u++) {
+                const float3 r = wrapped_difference(xj[u], x_row[row[u]], box);
+                if (ok[u]) out.store_vector(e0 + 256 * u, r);
+            }
+        }
+    }
+    for (int r = wave; r < nrows; r += 4)
+        if (rp[r + 1] - rp[r] > cap) refill_row(g, w, (int)(r0 + r), rp[r], capacity, out);
 }
 
 // order[k] = global id of the k-th atom in cell order (cells x-major, atoms by id inside a cell)
@@ -833,12 +1222,6 @@ __global__ void __launch_bounds__(256) padded_reduce_kernel(const int* __restric
     }
 }
 
-// torch's float `%` (floor-mod): fmod, then move a result of the wrong sign by one period
-__device__ __forceinline__ float floor_mod(float a, float b) {
-    float m = fmodf(a, b);
-    if (m != 0.f && ((b < 0.f) != (m < 0.f))) m += b;
-    return m;
-}
 
 __global__ void __launch_bounds__(256) edge_vectors_kernel(const float* __restrict__ x, const int* __restrict__ src,
                                                            const int* __restrict__ dst, long E, float bx, float by,
@@ -846,15 +1229,15 @@ __global__ void __launch_bounds__(256) edge_vectors_kernel(const float* __restri
                                                            int8_t* __restrict__ shift) {
     const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= E) return;
-    const long i = src[e], j = dst[e];
-    const float box[3] = {bx, by, bz};
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-        const float raw = x[3 * j + d] - x[3 * i + d];
-        const float half = 0.5f * box[d];
-        const float r = floor_mod(raw + half, box[d]) - half;
-        r_ij[3 * e + d] = r;
-        if (shift) shift[3 * e + d] = (int8_t)rintf(__fdiv_rn(raw - r, box[d]));
+    const float3 xi = load3(x + 3 * (long)src[e]), xj = load3(x + 3 * (long)dst[e]);
+    const float3 r = wrapped_difference(xj, xi, box_of(bx, by, bz));
+    r_ij[3 * e + 0] = r.x;
+    r_ij[3 * e + 1] = r.y;
+    r_ij[3 * e + 2] = r.z;
+    if (shift) {
+        shift[3 * e + 0] = (int8_t)rintf(__fdiv_rn((xj.x - xi.x) - r.x, bx));
+        shift[3 * e + 1] = (int8_t)rintf(__fdiv_rn((xj.y - xi.y) - r.y, by));
+        shift[3 * e + 2] = (int8_t)rintf(__fdiv_rn((xj.z - xi.z) - r.z, bz));
     }
 }
 
@@ -936,6 +1319,56 @@ int pairs_block_size(const Grid& g) {
     return mean_occ <= 2.0 ? 64 : 256;
 }
 
+
+// boxes small enough for box_search_kernel
+bool whole_box_search(const Grid& g) { return g.nodes <= kBoxNodes && g.ncells <= kBoxCells; }
+bool per_box_sort(const Grid& g) { return g.nodes <= kSortNodes && g.ncells <= kSortCells; }
+// words of box_max that the search leaves
+int box_max_entries(const Grid& g) { return whole_box_search(g) ? g.batch : per_box_sort(g) ? g.batch * sort_slabs(g) : 2; }
+
+template <int kPer, typename HitT>
+void launch_box_search(const float* x, const Grid& g, const Workspace& w, hipStream_t st) {
+    // workgroups per box: one home cell per wave while the whole search stays within two workgroups per CU
+    const int most = g.batch >= 512 ? 1 : 512 / g.batch;
+    int parts = (g.ncells + kBoxWaves - 1) / kBoxWaves;
+    parts = parts > most ? most : parts;
+    hipLaunchKernelGGL((box_search_kernel<kPer, HitT>), dim3((unsigned)parts, (unsigned)g.batch), dim3(kBoxThreads), 0, st, x,
+                       g, w);
+}
+
+// cell-ordered atoms, hit rows and degrees of every atom (batch * nodes > 0)
+int enqueue_search(const float* x, const Grid& g, const Workspace& w0, hipStream_t st) {
+    Workspace w = w0;
+    const long A = (long)g.batch * g.nodes, C = (long)g.batch * g.ncells;
+    if (whole_box_search(g)) {                     // (at most 2048 atoms per box: 16-bit hit rows)
+        if (g.nodes <= kBoxThreads) launch_box_search<1, unsigned short>(x, g, w, st);
+        else if (g.nodes <= 2 * kBoxThreads) launch_box_search<2, unsigned short>(x, g, w, st);
+        else launch_box_search<4, unsigned short>(x, g, w, st);
+        return check_launch("neighbour search");
+    }
+    const unsigned ablocks = (unsigned)ceil_div(A, 256);
+    if (per_box_sort(g)) {
+        hipLaunchKernelGGL(bin_kernel<false>, dim3(ablocks), dim3(256), 0, st, x, g, w);
+        hipLaunchKernelGGL(sort_box_kernel, dim3((unsigned)sort_slabs(g), (unsigned)g.batch), dim3(kSortThreads), 0, st, g, w);
+    } else {
+        hipLaunchKernelGGL(zero3_kernel, dim3((unsigned)(ceil_div(C, 256) < 1024 ? ceil_div(C, 256) : 1024)), dim3(256),
+                           0, st, w.box_max, 2L, (int*)nullptr, 0L, w.cell_count, C);
+        hipLaunchKernelGGL(bin_kernel<true>, dim3(ablocks), dim3(256), 0, st, x, g, w);
+        if (int s = run_scan(w.cell_count, C, w.cell_start, w, nullptr, w.box_max, nullptr, st)) return s;
+        hipLaunchKernelGGL(place_kernel, dim3(ablocks), dim3(256), 0, st, g, w);
+        hipLaunchKernelGGL(order_kernel, dim3(ablocks), dim3(256), 0, st, g, w);
+    }
+    const bool narrow = w.hit_bytes == 2;
+    if (pairs_block_size(g) == 64) {
+        if (narrow) hipLaunchKernelGGL((count_kernel<kCandCapSparse, unsigned short>), cell_grid(g), dim3(64), 0, st, g, w);
+        else hipLaunchKernelGGL((count_kernel<kCandCapSparse, int>), cell_grid(g), dim3(64), 0, st, g, w);
+    } else {
+        if (narrow) hipLaunchKernelGGL((count_kernel<kCandCapDense, unsigned short>), cell_grid(g), dim3(256), 0, st, g, w);
+        else hipLaunchKernelGGL((count_kernel<kCandCapDense, int>), cell_grid(g), dim3(256), 0, st, g, w);
+    }
+    return check_launch("neighbour search");
+}
+
 }  // namespace
 }  // namespace mg
 
@@ -968,7 +1401,7 @@ int mg_neighbour_count(const float* x, int batch, int nodes, float cutoff, float
     if (int s = make_grid(cutoff, box_x, box_y, box_z, batch, nodes, &g)) return s;
     MG_REQUIRE(row_ptr && stats && workspace, "mg_neighbour_count: null pointer");
     MG_REQUIRE(batch == 0 || edge_counts, "mg_neighbour_count: edge_counts is null");
-    const long A = (long)batch * nodes, C = (long)batch * g.ncells;
+    const long A = (long)batch * nodes;
     void* base = reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(workspace) + 255) & ~uintptr_t(255));
     Workspace w;
     size_t needed = 0;
@@ -981,34 +1414,13 @@ int mg_neighbour_count(const float* x, int batch, int nodes, float cutoff, float
         return check_launch("mg_neighbour_count");
     }
     MG_REQUIRE(x != nullptr, "mg_neighbour_count: x is null");
-    const unsigned ablocks = (unsigned)ceil_div(A, 256);
     const int deg_tiles = (int)ceil_div(A + 1, kScanTile);
-    const bool per_box_sort = nodes <= kSortNodes && g.ncells <= kSortCells;
-    if (per_box_sort) {
-        // six launches in all: bin, per-box sort, count, two for the scan of the degrees, fill
-        hipLaunchKernelGGL(bin_kernel<false>, dim3(ablocks), dim3(256), 0, st, x, g, w);
-        hipLaunchKernelGGL(sort_box_kernel, dim3((unsigned)sort_slabs(g), (unsigned)batch), dim3(kSortThreads), 0, st, g, w);
-    } else {
-        hipLaunchKernelGGL(zero3_kernel, dim3((unsigned)(ceil_div(C, 256) < 1024 ? ceil_div(C, 256) : 1024)), dim3(256),
-                           0, st, (int*)nullptr, 0L, row_ptr, 1L, w.cell_count, C);    // (every word of stats is stored below)
-        hipLaunchKernelGGL(bin_kernel<true>, dim3(ablocks), dim3(256), 0, st, x, g, w);
-        if (int s = run_scan(w.cell_count, C, w.cell_start, w, nullptr, stats + 1, nullptr, st)) return s;
-        hipLaunchKernelGGL(place_kernel, dim3(ablocks), dim3(256), 0, st, g, w);
-        hipLaunchKernelGGL(order_kernel, dim3(ablocks), dim3(256), 0, st, g, w);
-    }
-    const bool narrow = w.hit_bytes == 2;
-    if (pairs_block_size(g) == 64) {
-        if (narrow) hipLaunchKernelGGL((count_kernel<kCandCapSparse, unsigned short>), cell_grid(g), dim3(64), 0, st, g, w);
-        else hipLaunchKernelGGL((count_kernel<kCandCapSparse, int>), cell_grid(g), dim3(64), 0, st, g, w);
-    } else {
-        if (narrow) hipLaunchKernelGGL((count_kernel<kCandCapDense, unsigned short>), cell_grid(g), dim3(256), 0, st, g, w);
-        else hipLaunchKernelGGL((count_kernel<kCandCapDense, int>), cell_grid(g), dim3(256), 0, st, g, w);
-    }
+    if (int s = enqueue_search(x, g, w, st)) return s;
     hipLaunchKernelGGL(scan_sums_kernel, dim3((unsigned)deg_tiles), dim3(kScanThreads), 0, st, (const int*)w.degree, A,
                        w.deg_sums, w.deg_max);
     hipLaunchKernelGGL(scan_apply_kernel, dim3((unsigned)deg_tiles), dim3(kScanThreads), 0, st, (const int*)w.degree, A,
                        (const int*)w.deg_sums, (const int*)w.deg_max, deg_tiles, row_ptr, nodes, edge_counts, stats + 0,
-                       stats + 2, stats + 3, per_box_sort ? (const int*)w.box_max : (const int*)nullptr, batch * sort_slabs(g), stats + 1);
+                       stats + 2, stats + 3, (const int*)w.box_max, box_max_entries(g), stats + 1);
     return check_launch("mg_neighbour_count");
 }
 
@@ -1027,13 +1439,69 @@ int mg_neighbour_fill(const void* workspace, size_t workspace_bytes, int batch, 
     if (workspace_bytes == 0 || !layout(g, base, workspace_bytes, &w, &needed))
         return fail(MG_ERR_WORKSPACE, "mg_neighbour_fill: workspace has %zu bytes, at least %zu needed", workspace_bytes,
                     needed);
+    const EdgeOut out{src, dst, nullptr, nullptr, nullptr, nullptr};
     if (w.hit_bytes == 2)
         hipLaunchKernelGGL(fill_kernel<unsigned short>, dim3((unsigned)ceil_div(A, kFillRows)), dim3(256), 0,
-                           (hipStream_t)stream, g, w, row_ptr, src, dst, n_edges);
+                           (hipStream_t)stream, g, w, row_ptr, out, n_edges);
     else
         hipLaunchKernelGGL(fill_kernel<int>, dim3((unsigned)ceil_div(A, kFillRows)), dim3(256), 0, (hipStream_t)stream, g,
-                           w, row_ptr, src, dst, n_edges);
+                           w, row_ptr, out, n_edges);
     return check_launch("mg_neighbour_fill");
+}
+
+int mg_graph_search(const float* x, int batch, int nodes, float cutoff, float box_x, float box_y, float box_z,
+                    void* workspace, size_t workspace_bytes, mg_stream_t stream) {
+    Grid g;
+    if (int s = make_grid(cutoff, box_x, box_y, box_z, batch, nodes, &g)) return s;
+    if ((long)batch * nodes == 0) return MG_OK;
+    MG_REQUIRE(x && workspace, "mg_graph_search: null pointer");
+    void* base = reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(workspace) + 255) & ~uintptr_t(255));
+    Workspace w;
+    size_t needed = 0;
+    if (workspace_bytes == 0 || !layout(g, base, workspace_bytes, &w, &needed))
+        return fail(MG_ERR_WORKSPACE, "mg_graph_search: workspace has %zu bytes, at least %zu needed", workspace_bytes, needed);
+    hipStream_t st = (hipStream_t)stream;
+    if (int s = enqueue_search(x, g, w, st)) return s;
+    const long A = (long)batch * nodes;
+    if (A > kDirectRows)
+        hipLaunchKernelGGL(scan_sums_kernel, dim3((unsigned)ceil_div(A + 1, kScanTile)), dim3(kScanThreads), 0, st,
+                           (const int*)w.degree, A, w.deg_sums, w.deg_max);
+    return check_launch("mg_graph_search");
+}
+
+int mg_graph_fill(const float* x, const void* workspace, size_t workspace_bytes, int batch, int nodes, float cutoff,
+                  float box_x, float box_y, float box_z, int* row_ptr, int* edge_counts, int* stats, int capacity, int* src,
+                  int* dst, int64_t* src64, int64_t* dst64, float* r_ij, int* order, mg_stream_t stream) {
+    Grid g;
+    if (int s = make_grid(cutoff, box_x, box_y, box_z, batch, nodes, &g)) return s;
+    MG_REQUIRE(capacity >= 0, "mg_graph_fill: negative capacity");
+    MG_REQUIRE(row_ptr && stats, "mg_graph_fill: null pointer");
+    MG_REQUIRE((src64 == nullptr) == (dst64 == nullptr), "mg_graph_fill: src64 and dst64 go together");
+    const long A = (long)batch * nodes;
+    hipStream_t st = (hipStream_t)stream;
+    if (A == 0) {
+        hipLaunchKernelGGL(zero3_kernel, dim3(1), dim3(256), 0, st, stats, 4L, row_ptr, 1L, edge_counts, (long)batch);
+        return check_launch("mg_graph_fill");
+    }
+    MG_REQUIRE(workspace && edge_counts && (capacity == 0 || (src && dst)) && (r_ij == nullptr || x),
+               "mg_graph_fill: null pointer");
+    void* base = reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(workspace) + 255) & ~uintptr_t(255));
+    Workspace w;
+    size_t needed = 0;
+    if (workspace_bytes == 0 || !layout(g, base, workspace_bytes, &w, &needed))
+        return fail(MG_ERR_WORKSPACE, "mg_graph_fill: workspace has %zu bytes, at least %zu needed", workspace_bytes, needed);
+    const EdgeOut out{src, dst, src64, dst64, r_ij, x};
+    // few rows: workgroups of 8, so that a small graph still spreads over the chip
+    const int rows_per = A <= 4096 ? 8 : kFillRows;
+    const dim3 grid((unsigned)ceil_div(A, rows_per));
+    const int tiled = A > kDirectRows ? 1 : 0;
+    if (w.hit_bytes == 2)
+        hipLaunchKernelGGL(graph_fill_kernel<unsigned short>, grid, dim3(256), 0, st, g, w, rows_per, tiled,
+                           box_max_entries(g), row_ptr, edge_counts, stats, capacity, out, order);
+    else
+        hipLaunchKernelGGL(graph_fill_kernel<int>, grid, dim3(256), 0, st, g, w, rows_per, tiled, box_max_entries(g), row_ptr,
+                           edge_counts, stats, capacity, out, order);
+    return check_launch("mg_graph_fill");
 }
 
 int mg_neighbour_edges(const float* x, int batch, int nodes, float cutoff, float box_x, float box_y, float box_z,

@@ -14,8 +14,13 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
+#include <algorithm>
 #include <array>
+#include <atomic>
+#include <chrono>
 #include <cstdint>
+#include <map>
+#include <mutex>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -103,11 +108,11 @@ Search count_phase(float cutoff, float bx, float by, float bz, const at::Tensor&
 }
 
 // the reference's overflow errors, in the reference's order (neighbour_grid_kern.cu:195-217)
-void check_caps(const Search& s, int listmax, int neighboursmax) {
-    TORCH_CHECK(s.stats[1] <= listmax, "Cell list overflow occurred. Trying increasing listmax.");
+void check_caps(const int* stats, int listmax, int neighboursmax) {
+    TORCH_CHECK(stats[1] <= listmax, "Cell list overflow occurred. Trying increasing listmax.");
     TORCH_CHECK(listmax == 32 || listmax == 64 || listmax == 128 || listmax == 256,
                 "expected listmax to be one of 32, 64, 128, 256. other values not supported!");
-    TORCH_CHECK(s.stats[2] <= neighboursmax, "Neighbour list overflow occurred. Try increasing neighboursmax.");
+    TORCH_CHECK(stats[2] <= neighboursmax, "Neighbour list overflow occurred. Try increasing neighboursmax.");
 }
 
 std::pair<at::Tensor, at::Tensor> fill_phase(const Search& s, float cutoff, float bx, float by, float bz,
@@ -125,7 +130,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> get_edges(int listmax, int neighb
     check_input(x, "x");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     const Search s = count_phase(cutoff, bx, by, bz, x);
-    check_caps(s, listmax, neighboursmax);
+    check_caps(s.stats, listmax, neighboursmax);
     auto edges = fill_phase(s, cutoff, bx, by, bz, x);
     return {edges.first, edges.second, s.edge_counts};
 }
@@ -135,7 +140,7 @@ std::tuple<at::Tensor, at::Tensor> get_neighbours(int listmax, int neighboursmax
     check_input(x, "x");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     const Search s = count_phase(cutoff, bx, by, bz, x);
-    check_caps(s, listmax, neighboursmax);
+    check_caps(s.stats, listmax, neighboursmax);
     auto edges = fill_phase(s, cutoff, bx, by, bz, x);
     const int batch = (int)x.size(0), nodes = (int)x.size(1);
     const auto i32 = x.options().dtype(at::kInt);
@@ -143,6 +148,112 @@ std::tuple<at::Tensor, at::Tensor> get_neighbours(int listmax, int neighboursmax
     check(mg_neighbour_pad(s.row_ptr.data_ptr<int>(), edges.second.data_ptr<int>(), batch, nodes, neighboursmax,
                            neighbours.data_ptr<int>(), counts.data_ptr<int>(), stream_of(x)));
     return {neighbours, counts};
+}
+
+// The radius graph of Graph.radius_graph / graph_setup in one call.  The fill pass is queued before the edge count is
+// known, into arrays sized from an estimate (the count of the last search of this shape, else the mean density, plus a
+// margin), while the host polls the four statistics, which the kernel stores into pinned memory; only an estimate that
+// was too small costs a second pass.
+struct PinnedWords {                                   // four int32 words the device writes and the host polls
+    std::mutex mutex;
+    std::vector<at::Tensor> free;
+    at::Tensor take() {
+        std::lock_guard<std::mutex> lock(mutex);
+        if (free.empty()) return at::empty({4}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+        at::Tensor t = free.back();
+        free.pop_back();
+        return t;
+    }
+    void give(const at::Tensor& t) {                   // (after every word has arrived: nothing will write them again)
+        std::lock_guard<std::mutex> lock(mutex);
+        if (free.size() < 64) free.push_back(t);
+    }
+};
+PinnedWords& pinned_words() {
+    static PinnedWords* pool = new PinnedWords;        // never destroyed: the allocator may be gone by then
+    return *pool;
+}
+
+struct EdgeHints {                                     // edge count of the last search of a shape
+    using Key = std::tuple<int, int, float, float, float, float>;
+    std::mutex mutex;
+    std::map<Key, int> counts;
+    int64_t get(const Key& k, int64_t otherwise) {
+        std::lock_guard<std::mutex> lock(mutex);
+        auto it = counts.find(k);
+        return it == counts.end() ? otherwise : it->second;
+    }
+    void put(const Key& k, int n) {
+        std::lock_guard<std::mutex> lock(mutex);
+        if (counts.size() > 256) counts.clear();
+        counts[k] = n;
+    }
+};
+EdgeHints& edge_hints() {
+    static EdgeHints* hints = new EdgeHints;
+    return *hints;
+}
+
+// (src, dst, src64, dst64, edge_counts, row_ptr, order, r_ij or None), or None when a coordinate is NaN
+py::object radius_graph(int listmax, int neighboursmax, float cutoff, float bx, float by, float bz, const at::Tensor& x,
+                        bool want_vectors) {
+    check_input(x, "x");
+    TORCH_CHECK(x.dim() == 3 && x.size(2) == 3, "x must have shape (batch, nodes, 3)");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    const int batch = (int)x.size(0), nodes = (int)x.size(1);
+    const int64_t atoms = (int64_t)batch * nodes;
+    size_t bytes = 0;
+    check(mg_neighbour_workspace_bytes(batch, nodes, cutoff, bx, by, bz, &bytes));
+    const auto i32 = x.options().dtype(at::kInt), i64 = x.options().dtype(at::kLong);
+    at::Tensor workspace = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
+    at::Tensor row_ptr = at::empty({atoms + 1}, i32), edge_counts = at::empty({batch}, i32), order = at::empty({atoms}, i32);
+    const mg_stream_t stream = stream_of(x);
+    check(mg_graph_search(fp(x), batch, nodes, cutoff, bx, by, bz, workspace.data_ptr(), bytes, stream));
+    const EdgeHints::Key key{batch, nodes, cutoff, bx, by, bz};
+    const double mean = atoms > 0 ? 1.5 * atoms * (nodes / ((double)bx * by * bz)) * 4.18879 * cutoff * cutoff * cutoff : 0.0;
+    int64_t capacity = (int64_t)(1.125 * edge_hints().get(key, (int64_t)std::min(mean, 2e9))) + 4096;
+    capacity = std::min<int64_t>(capacity, 0x7fffffff);
+    at::Tensor src, dst, src64, dst64, r_ij;
+    at::Tensor words = pinned_words().take();
+    volatile int* w = words.data_ptr<int>();
+    int st[4] = {0, 0, 0, 0};
+    for (int attempt = 0;; attempt++) {
+        src = at::empty({capacity}, i32);
+        dst = at::empty({capacity}, i32);
+        src64 = at::empty({capacity}, i64);
+        dst64 = at::empty({capacity}, i64);
+        if (want_vectors) r_ij = at::empty({capacity, 3}, x.options());
+        for (int k = 0; k < 4; k++) w[k] = -1;         // (never a valid value)
+        check(mg_graph_fill(fp(x), workspace.data_ptr(), bytes, batch, nodes, cutoff, bx, by, bz, row_ptr.data_ptr<int>(),
+                            edge_counts.data_ptr<int>(), words.data_ptr<int>(), (int)capacity, src.data_ptr<int>(),
+                            dst.data_ptr<int>(), src64.data_ptr<int64_t>(), dst64.data_ptr<int64_t>(),
+                            want_vectors ? fp(r_ij) : nullptr, order.data_ptr<int>(), stream));
+        {
+            py::gil_scoped_release release;
+            auto arrived = [&] { return w[0] >= 0 && w[1] >= 0 && w[2] >= 0 && w[3] >= 0; };
+            const auto began = std::chrono::steady_clock::now();
+            for (long polls = 0; !arrived(); polls++) {
+                if ((polls & 1023) == 1023 && std::chrono::steady_clock::now() - began > std::chrono::milliseconds(50)) {
+                    c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.device().index()).synchronize();
+                    break;
+                }
+            }
+            std::atomic_thread_fence(std::memory_order_acquire);
+        }
+        for (int k = 0; k < 4; k++) st[k] = w[k];
+        TORCH_CHECK(st[0] >= 0 && st[1] >= 0 && st[2] >= 0 && st[3] >= 0, "the neighbour search did not report its statistics");
+        if (st[0] <= capacity || (st[3] & 5)) break;
+        TORCH_CHECK(attempt == 0, "the edge count changed between two fill passes");
+        capacity = st[0];
+    }
+    pinned_words().give(words);
+    if (st[3] & 4) return py::none();
+    TORCH_CHECK((st[3] & 1) == 0, "edge count does not fit int32");
+    edge_hints().put(key, st[0]);
+    check_caps(st, listmax, neighboursmax);
+    const int64_t E = st[0];
+    return py::make_tuple(src.narrow(0, 0, E), dst.narrow(0, 0, E), src64.narrow(0, 0, E), dst64.narrow(0, 0, E), edge_counts,
+                          row_ptr, order, want_vectors ? py::cast(r_ij.narrow(0, 0, E)) : py::none());
 }
 
 at::Tensor edges_read(const at::Tensor& counts, const at::Tensor& neighbours, const at::Tensor& x) {
@@ -420,6 +531,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("edges_read", &edges_read, "Read data from nodes to edges.");
     m.def("edges_reduce", &edges_reduce, "Reduce data from edges to nodes.");
     m.def("get_edges", &get_edges, "Like get_neighbours, except it returns lists of edge tensors.");
+    // Graph.radius_graph and graph_setup (managan/graph_layers.py:25-34,62-66)
+    m.def("radius_graph", &radius_graph);
     // tensor_ops_cuda (tensor_ops.cpp:180-182)
     m.def("tensor_linear", &tensor_linear, "tensor_linear(inds, W, x)");
     // TensorProds.forward (managan/tensor_products.py:109-121) as one launch

@@ -13,6 +13,7 @@ as taken by torch.autograd.functional.jvp(create_graph=True) work too).
 """
 import torch
 
+from . import _lib as L
 from . import ops
 
 
@@ -21,11 +22,11 @@ class Graph:
     and index into a dimension of size batch*nodes.  src must be non-decreasing.
     (managan/graph_layers.py:9-24)"""
 
-    def __init__(self, src, dst, edge_indices, batch, nodes, row_ptr=None, cell_order=None):
+    def __init__(self, src, dst, edge_indices, batch, nodes, row_ptr=None, cell_order=None, wide=None):
+        """wide: (src, dst) as int64, when the caller holds them in both widths."""
         self.src32 = src.to(torch.int32).contiguous()
         self.dst32 = dst.to(torch.int32).contiguous()
-        self.src = src.to(torch.int64)
-        self.dst = dst.to(torch.int64)
+        self.src, self.dst = (src.to(torch.int64), dst.to(torch.int64)) if wide is None else wide
         self.edge_indices = edge_indices
         self.batch = batch
         self.nodes = nodes
@@ -68,14 +69,20 @@ class Graph:
         """Nodes are connected if they are within r0 of each other under periodic
         boundary conditions given by box (3 floats).  pos: (batch, nodes, 3).
         (managan/graph_layers.py:25-34)"""
-        batch, nodes, three = pos.shape
-        assert three == 3
-        assert torch.all(~torch.isnan(pos)), "some positions are NaN!"
-        src, dst, edge_indices, row_ptr, order = ops.get_edges(celllist_max, neighbours_max, r0, *box, pos,
-                                                               return_row_ptr=True, return_order=True)
-        ans = Graph(src, dst, edge_indices, batch, nodes, row_ptr=row_ptr, cell_order=order)
-        setattr(ans, "box", box)
-        return ans
+        return _search(r0, box, pos, celllist_max, neighbours_max, False)[0]
+
+
+def _search(r0, box, pos, celllist_max, neighbours_max, want_vectors):
+    """The radius graph and, with want_vectors, its edge vectors, from the same kernel."""
+    batch, nodes, three = pos.shape
+    assert three == 3
+    found = L.load_torch_ext().radius_graph(celllist_max, neighbours_max, r0, *(float(b) for b in box), pos,
+                                            want_vectors)
+    assert found is not None, "some positions are NaN!"
+    src, dst, src64, dst64, edge_indices, row_ptr, order, r_ij = found
+    ans = Graph(src, dst, edge_indices, batch, nodes, row_ptr=row_ptr, cell_order=order, wide=(src64, dst64))
+    setattr(ans, "box", box)
+    return ans, r_ij
 
 
 class _SortedIndex:
@@ -190,8 +197,7 @@ def edge_vectors(graph: Graph, pos: torch.Tensor, box, want_shift=False):
 
 
 def graph_setup(r0, box, pos, neighbours_max=64, celllist_max=32):
-    graph = Graph.radius_graph(r0, box, pos, celllist_max=celllist_max, neighbours_max=neighbours_max)
-    return graph, edge_vectors(graph, pos, box)
+    return _search(r0, box, pos, celllist_max, neighbours_max, True)
 
 
 def graph_setup_capacity(r0, box, pos, capacity, buffers=None):

@@ -326,3 +326,48 @@ def test_workspace_smaller_than_the_preferred_size(nodes, box_len, cutoff):
             assert torch.equal(a, b)
     status, _ = search(fixed + A * 31 * entry)
     assert status == L.MG_ERR_WORKSPACE and b"at least" in lib.mg_last_error()
+
+
+# the one-kernel search takes boxes of at most 2048 atoms (512 threads, 1, 2 or 4 atoms each) and 4096 cells; the fill pass
+# adds degrees up directly to 16384 rows; 20000 atoms leave the per-box sort; the last two boxes hold more than 64 atoms per
+# cell and more neighbours than a hit row has entries
+@pytest.mark.parametrize("batch,atoms,side,cutoff,spread", [
+    (1, 1, 16., 5., 1.), (3, 2, 16., 5., 1.), (1, 511, 16., 5., 1.), (2, 513, 17., 5., 1.), (1, 1025, 22., 5., 1.),
+    (9, 2048, 27.4, 6., 1.), (1, 2049, 27.5, 5., 1.), (1, 2048, 90., 5., 1.), (1, 16384, 55., 5., 1.), (3, 5462, 38., 5., 1.),
+    (1, 20000, 60., 5., 1.), (2, 700, 40., 6., 0.25), (1, 3000, 40., 6., 0.45)])
+def test_graph_setup_against_the_oracle(pkg, batch, atoms, side, cutoff, spread):
+    """graph_setup (search, int64 indices, edge vectors and cell order from the fused kernels): sorted edges, counts, row
+    pointer and edge vectors bit for bit."""
+    gl = importlib.import_module("learned-dynamics_amd.graph_layers")
+    rng = np.random.default_rng(atoms + batch)
+    box = (side, side * 1.01, side * 1.02)
+    x = (rng.random((batch, atoms, 3)) * spread * np.array(box) + rng.integers(-2, 3, (batch, atoms, 3)) * np.array(box))
+    x = x.astype(np.float32)
+    graph, r_ij = gl.graph_setup(cutoff, box, torch.from_numpy(x).cuda(), neighbours_max=100000, celllist_max=256) \
+        if spread == 1. else (None, None)
+    if graph is None:                # crowded cells: past the reference's caps, which graph_setup raises on
+        with pytest.raises(RuntimeError, match="overflow"):
+            gl.graph_setup(cutoff, box, torch.from_numpy(x).cuda(), neighbours_max=64, celllist_max=32)
+        ext = importlib.import_module("learned-dynamics_amd._lib").load_torch_ext()
+        found = ext.radius_graph(256, 100000, cutoff, *box, torch.from_numpy(x).cuda(), True)
+        src32, dst32, src, dst, counts, row_ptr, order, r_ij = found
+    else:
+        src32, dst32, src, dst, counts, row_ptr, order = (graph.src32, graph.dst32, graph.src, graph.dst, graph.edge_indices,
+                                                          graph.row_ptr, graph.cell_order)
+    ref = ON.edges(x, cutoff, box, ON.MODE_CELLS)
+    s, d = src.cpu().numpy(), dst.cpu().numpy()
+    assert torch.equal(src32.long(), src) and torch.equal(dst32.long(), dst)
+    np.testing.assert_array_equal(counts.cpu().numpy(), ref["edge_counts"])
+    np.testing.assert_array_equal(np.diff(row_ptr.cpu().numpy()), ref["counts"].reshape(-1))
+    np.testing.assert_array_equal(_triples(s, d), _triples(ref["src"], ref["dst"]))
+    np.testing.assert_array_equal(r_ij.cpu().numpy(), ON.edge_vectors(x, s, d, box))
+    assert torch.equal(order.sort().values, torch.arange(batch * atoms, device="cuda", dtype=torch.int32))
+
+
+@pytest.mark.parametrize("atoms", [300, 5000, 20000])
+def test_graph_setup_rejects_nan(pkg, atoms):
+    gl = importlib.import_module("learned-dynamics_amd.graph_layers")
+    x = torch.rand(2, atoms, 3, device="cuda") * 60
+    x[1, atoms // 2, 1] = float("nan")
+    with pytest.raises(AssertionError, match="NaN"):
+        gl.graph_setup(5.0, (60., 60., 60.), x, neighbours_max=1000, celllist_max=256)
