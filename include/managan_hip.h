@@ -317,8 +317,14 @@ int mg_tensor_linear_packed(const void* packed_W, const float* x, long rows, int
 int mg_linear_f16x2_packed_weight_bytes(int dim_in, int dim_out, size_t* bytes /* host */);
 int mg_linear_f16x2_pack_weight(const float* W, long w_stride_o, long w_stride_i, int dim_in, int dim_out,
                                 void* packed, mg_stream_t stream);
+/* the same with zero columns appended up to dim_pad (a multiple of 32): the packed weight of a reduction that long */
+int mg_linear_f16x2_pack_weight_padded(const float* W, long w_stride_o, long w_stride_i, int dim_in, int dim_out, int dim_pad,
+                                       void* packed, mg_stream_t stream);
 int mg_row_absmax(const float* x, long rows, int dim, float* out /* (rows) */, mg_stream_t stream);
-int mg_tensor_linear_f16x2_rowmax_parts(long rows, int dim_in, int dim_out);   /* returns the count, not a status */
+int mg_tensor_linear_f16x2_rowmax_parts(long rows, int dim_in, int dim_out);
+/* 1 when mg_tensor_linear_f16x2 splits the reduction of a problem of this size over the waves of a workgroup (few rows)
+ * instead of streaming rows; a caller that wants the rows' sums per segment then takes the product and a segment sum. */
+int mg_tensor_linear_f16x2_splits_k(long rows, int dim_in, int dim_out);   /* returns the count, not a status */
 int mg_tensor_linear_f16x2(const void* packed_W, const float* x, const float* x_rowmax, int x_rowmax_parts,
                            long x_rowmax_stride, long x_rows_per_bound, long rows, int dim_in, int dim_out, const float* bias, int act, int accumulate,
                            int out_comps, float* y, float* y_rowmax, mg_stream_t stream);
@@ -329,6 +335,28 @@ int mg_tensor_linear_f16x2_scaled_bound(const void* packed_W, const float* x, co
                                         long x_rowmax_stride, long x_rows_per_bound, long rows, int dim_in, int dim_out,
                                         const float* bias, int act, int accumulate, int out_comps, float* y,
                                         float* y_rowmax, float bound_mul, float bound_add, mg_stream_t stream);
+/* The same with every option as a field.  bias_rows: rows from this one on get no bias (the tangents stacked behind the
+ * values of a forward-mode pass; then act = 0, accumulate = 0, out_comps = 1); rows or more: all rows.  sequential != 0:
+ * the reduction of an output element runs over k in order whatever the number of rows is, so a row's result does not
+ * depend on the batch it is in, bit for bit (few rows otherwise split the reduction); y_rowmax then has
+ * mg_tensor_linear_f16x2_rowmax_parts_sequential parts. */
+typedef struct mg_f16x2_linear {
+    const void* packed_W;
+    const float* x;
+    const float* x_rowmax;
+    int x_rowmax_parts;
+    long x_rowmax_stride, x_rows_per_bound;
+    float bound_mul, bound_add;
+    long rows;
+    int dim_in, dim_out;
+    const float* bias;
+    long bias_rows;
+    int act, accumulate, out_comps, sequential;
+    float* y;
+    float* y_rowmax;
+} mg_f16x2_linear;
+int mg_tensor_linear_f16x2_run(const mg_f16x2_linear* args /* host */, mg_stream_t stream);
+int mg_tensor_linear_f16x2_rowmax_parts_sequential(long rows, int dim_in, int dim_out);
 /* y = act(x W^T + bias) in float64 arithmetic: W (dim_out, dim_in) and bias are the float32 parameters, widened
  * exactly; x (rows, dim_in), every product and sum, the activation and y (rows, dim_out) are double.  The same
  * contraction as nn.Linear inside the reference's MLPs (archs/meanflow_painn8.py:38-51); float64 has no counterpart

@@ -78,6 +78,10 @@ _SIGNATURES = {
     "mg_linear_f16x2_pack_weight": [vp, i64, i64, i32, i32, vp, vp],
     "mg_row_absmax": [vp, i64, i32, vp, vp],
     "mg_linear_f64": [vp, vp, vp, i64, i32, i32, i32, vp, vp],
+    "mg_tensor_linear_f16x2_run": [vp, vp],
+    "mg_tensor_linear_f16x2_rowmax_parts_sequential": [i64, i32, i32],
+    "mg_linear_f16x2_pack_weight_padded": [vp, i64, i64, i32, i32, i32, vp, vp],
+    "mg_tensor_linear_f16x2_splits_k": [i64, i32, i32],
     "mg_tensor_linear_f16x2_rowmax_parts": [i64, i32, i32],
     "mg_tensor_linear_f16x2": [vp, vp, vp, i32, i64, i64, i64, i32, i32, vp, i32, i32, i32, vp, vp, vp],
     "mg_tensor_linear_f16x2_scaled_bound": [vp, vp, vp, i32, i64, i64, i64, i32, i32, vp, i32, i32, i32, vp, vp,

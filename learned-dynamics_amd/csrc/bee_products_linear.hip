@@ -60,7 +60,7 @@ products_linear_kernel(const _Float16* __restrict__ Wp, const float* __restrict_
                        const float* __restrict__ node_bound, long n_nodes, int chan, int O, int O_pad,
                        float* __restrict__ Y, int tiles_n, long tiles_total) {
     constexpr int TM = 32 * WAVES, TN = 32 * NI, THREADS = 64 * WAVES;
-    constexpr int kPlaneW = TN * kRowW, kBufW = 2 * kPlaneW;
+    constexpr int kPlaneW = TN * 64, kBufW = 2 * kPlaneW;
     constexpr int kPieces = 8 * TN;
     constexpr int kPer = (kPieces + THREADS - 1) / THREADS;
     __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kBufW];
@@ -105,9 +105,9 @@ products_linear_kernel(const _Float16* __restrict__ Wp, const float* __restrict_
     for (int j = 0; j < kPer; j++) {
         int q = tid + THREADS * j;
         if (q >= kPieces) q = kPieces - 1;
-        const int plane = q / (4 * TN), row = (q % (4 * TN)) >> 2, piece = q & 3;
-        wsrc[j] = Wp + plane * plane_elems + (long)(n0 + row) * I + 8 * piece;
-        wdst[j] = plane * kPlaneW + row * kRowW + piece * 16;
+        const int plane = q / (4 * TN), i = q % (4 * TN);
+        wsrc[j] = Wp + plane * plane_elems + packed_piece(n0, i, I);
+        wdst[j] = plane * kPlaneW + 16 * i;
     }
     const int k_last = I - kCK;
 
@@ -146,13 +146,13 @@ products_linear_kernel(const _Float16* __restrict__ Wp, const float* __restrict_
     auto load_w = [&](WRegs& w, int k0) {
         k0 = k0 < I ? k0 : k_last;
 #pragma unroll
-        for (int j = 0; j < kPer; j++) w.v[j] = *reinterpret_cast<const halfx8*>(wsrc[j] + k0);
+        for (int j = 0; j < kPer; j++) w.v[j] = *reinterpret_cast<const halfx8*>(wsrc[j] + 32L * k0);
     };
     auto store_w = [&](const WRegs& w, unsigned char* buf) {
 #pragma unroll
         for (int j = 0; j < kPer; j++) *reinterpret_cast<halfx8*>(buf + wdst[j]) = w.v[j];
     };
-    const int b_off = m * kRowW + 32 * g;
+    const int b_off = 16 * lane;
     auto compute = [&](const ARegs& a, const unsigned char* buf, float scale) {
         halfx8 ah[2], al[2];
 #pragma unroll
@@ -168,8 +168,8 @@ products_linear_kernel(const _Float16* __restrict__ Wp, const float* __restrict_
         for (int s = 0; s < 2; s++)
 #pragma unroll
             for (int ni = 0; ni < NI; ni++) {
-                const halfx8 bh = *reinterpret_cast<const halfx8*>(buf + b_off + ni * 32 * kRowW + 16 * s);
-                const halfx8 bl = *reinterpret_cast<const halfx8*>(buf + kPlaneW + b_off + ni * 32 * kRowW + 16 * s);
+                const halfx8 bh = *reinterpret_cast<const halfx8*>(buf + b_off + 2048 * ni + 1024 * s);
+                const halfx8 bl = *reinterpret_cast<const halfx8*>(buf + kPlaneW + b_off + 2048 * ni + 1024 * s);
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[s], bh, acc[ni], 0, 0, 0);
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s], bl, acc[ni], 0, 0, 0);
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s], bh, acc[ni], 0, 0, 0);
@@ -234,7 +234,7 @@ products_linear_staged_kernel(const _Float16* __restrict__ Wp, const float* __re
     constexpr int T = 9, WAVES = 4, TM = 32 * WAVES, TN = 32 * NI, THREADS = 64 * WAVES;
     constexpr int NN = TM / T + 2;                           // nodes a tile of TM rows can touch
     constexpr int kRowF = 36;                                // floats per staged row: 32 channels + 4 (bank spread)
-    constexpr int kPlaneW = TN * kRowW, kBufW = 2 * kPlaneW;
+    constexpr int kPlaneW = TN * 64, kBufW = 2 * kPlaneW;
     constexpr int kPieces = 8 * TN;
     constexpr int kPer = (kPieces + THREADS - 1) / THREADS;
     __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kBufW];
@@ -281,9 +281,9 @@ products_linear_staged_kernel(const _Float16* __restrict__ Wp, const float* __re
     for (int j = 0; j < kPer; j++) {
         int q = tid + THREADS * j;
         if (q >= kPieces) q = kPieces - 1;
-        const int plane = q / (4 * TN), row = (q % (4 * TN)) >> 2, piece = q & 3;
-        wsrc[j] = Wp + plane * plane_elems + (long)(n0 + row) * I + 8 * piece;
-        wdst[j] = plane * kPlaneW + row * kRowW + piece * 16;
+        const int plane = q / (4 * TN), i = q % (4 * TN);
+        wsrc[j] = Wp + plane * plane_elems + packed_piece(n0, i, I);
+        wdst[j] = plane * kPlaneW + 16 * i;
     }
     const int k_last = I - kCK;
     struct ARegs { float4 v[4]; };
@@ -343,13 +343,13 @@ products_linear_staged_kernel(const _Float16* __restrict__ Wp, const float* __re
     auto load_w = [&](WRegs& w, int k0) {
         k0 = k0 < I ? k0 : k_last;
 #pragma unroll
-        for (int j = 0; j < kPer; j++) w.v[j] = *reinterpret_cast<const halfx8*>(wsrc[j] + k0);
+        for (int j = 0; j < kPer; j++) w.v[j] = *reinterpret_cast<const halfx8*>(wsrc[j] + 32L * k0);
     };
     auto store_w = [&](const WRegs& w, unsigned char* buf) {
 #pragma unroll
         for (int j = 0; j < kPer; j++) *reinterpret_cast<halfx8*>(buf + wdst[j]) = w.v[j];
     };
-    const int b_off = m * kRowW + 32 * g;
+    const int b_off = 16 * lane;
     auto compute = [&](const ARegs& a, const unsigned char* buf) {
         halfx8 ah[2], al[2];
 #pragma unroll
@@ -365,8 +365,8 @@ products_linear_staged_kernel(const _Float16* __restrict__ Wp, const float* __re
         for (int s = 0; s < 2; s++)
 #pragma unroll
             for (int ni = 0; ni < NI; ni++) {
-                const halfx8 bh = *reinterpret_cast<const halfx8*>(buf + b_off + ni * 32 * kRowW + 16 * s);
-                const halfx8 bl = *reinterpret_cast<const halfx8*>(buf + kPlaneW + b_off + ni * 32 * kRowW + 16 * s);
+                const halfx8 bh = *reinterpret_cast<const halfx8*>(buf + b_off + 2048 * ni + 1024 * s);
+                const halfx8 bl = *reinterpret_cast<const halfx8*>(buf + kPlaneW + b_off + 2048 * ni + 1024 * s);
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[s], bh, acc[ni], 0, 0, 0);
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s], bl, acc[ni], 0, 0, 0);
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s], bh, acc[ni], 0, 0, 0);

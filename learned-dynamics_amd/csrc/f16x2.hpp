@@ -39,6 +39,19 @@ __device__ __forceinline__ HalfSplit4 split(float4 v, float s) {
 }
 
 constexpr int kCK = 32;                     // k per chunk (two MFMA steps)
-constexpr int kRowW = 80;                   // bytes per LDS row of one W plane (64 + 16 pad)
+
+// Packed planes of a weight (O, I): in the order the matrix cores read them.  A block of 32 output rows x one chunk of 32
+// k is 1024 halves: step s of the chunk (512 halves), lane = row % 32 + 32 g of the fragment, its 8 consecutive
+// k = 32 c + 16 g + 8 s .. + 8.  Blocks of rows outermost, then chunks.  A wave's fragment load is one contiguous
+// kilobyte, from memory or from LDS (no padding, no bank conflicts); in row-major planes the 64 lanes of such a load sat in
+// 32 rows and the vector-memory front end took them line by line.
+__host__ __device__ __forceinline__ long packed_index(long o, int k, int I) {
+    return ((o >> 5) * (I >> 5) + (k >> 5)) * 1024L + ((k >> 3) & 1) * 512 + ((((k >> 4) & 1) << 5) + (o & 31)) * 8 + (k & 7);
+}
+// the i-th 16-byte piece (i = 128 block + 64 s + lane) of chunk 0 of a tile of output rows that starts at n0 (a multiple
+// of 32); chunk k0 / 32 of the same piece is kPackedChunk * (k0 / 32) = 32 k0 halves further on
+__device__ __forceinline__ long packed_piece(int n0, int i, int I) {
+    return ((long)((n0 >> 5) + (i >> 7)) * (I >> 5)) * 1024L + (i & 127) * 8;
+}
 
 }  // namespace mg

@@ -45,10 +45,11 @@ __device__ __forceinline__ float activate_c(float v) {
 }
 
 constexpr int kFThreads = 64 * kFW;
-constexpr int kFPlaneW = kFTN * kRowW, kFBufW = 2 * kFPlaneW;   // bytes of one W plane / of both planes of a chunk
-constexpr int kFSlice = 2 * kFBufW / kFW / 4;                    // floats of LDS per wave once the main loop is over
+constexpr int kFPlaneW = kFTN * 64, kFBufW = 2 * kFPlaneW;   // bytes of one W plane / of both planes of a chunk
 constexpr int kFRed = 68;                                        // floats per row of a slice: 64 + 4 (spreads 16-byte writes over the banks)
-static_assert(kFSlice >= 32 * kFRed, "a reduction pass needs 32 rows x 64 columns per wave");
+constexpr int kFSlice = 32 * kFRed;                              // floats of LDS per wave once the main loop is over: a
+                                                                 // reduction pass has 32 rows x 64 columns per wave
+constexpr int kFLds = 2 * kFBufW > 4 * kFW * kFSlice ? 2 * kFBufW : 4 * kFW * kFSlice;
 
 // Source of the second operand: the 16 values x[row][k0 + 16 g ..] of this lane's row for chunk k0, from memory
 struct RowFromMemory {
@@ -74,15 +75,14 @@ __device__ __forceinline__ void wfirst_gemm_tile(floatx16 (&acc)[kFNI], const _F
     constexpr int THREADS = kFThreads, kPlaneW = kFPlaneW, kBufW = kFBufW;
     constexpr int kPer = 8 * kFTN / THREADS;                 // 16-byte pieces of W per thread and chunk
     const int tid = threadIdx.x;
-    const int m = tid & 31, g = (tid >> 5) & 1;
     const _Float16* wsrc[kPer];
     int wdst[kPer];
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
         const int q = tid + THREADS * j;
-        const int plane = q / (4 * kFTN), row = (q % (4 * kFTN)) >> 2, piece = q & 3;
-        wsrc[j] = Wp + plane * plane_elems + (long)(n0 + row) * I + 8 * piece;
-        wdst[j] = plane * kPlaneW + row * kRowW + piece * 16;
+        const int plane = q / (4 * kFTN), i = q % (4 * kFTN);
+        wsrc[j] = Wp + plane * plane_elems + packed_piece(n0, i, I);
+        wdst[j] = plane * kPlaneW + 16 * i;
     }
     const int k_last = I - kCK;
 
@@ -92,13 +92,13 @@ __device__ __forceinline__ void wfirst_gemm_tile(floatx16 (&acc)[kFNI], const _F
     auto load_w = [&](WRegs& w, int k0) {
         k0 = k0 < I ? k0 : k_last;
 #pragma unroll
-        for (int j = 0; j < kPer; j++) w.v[j] = *reinterpret_cast<const halfx8*>(wsrc[j] + k0);
+        for (int j = 0; j < kPer; j++) w.v[j] = *reinterpret_cast<const halfx8*>(wsrc[j] + 32L * k0);
     };
     auto store_w = [&](const WRegs& w, unsigned char* buf) {
 #pragma unroll
         for (int j = 0; j < kPer; j++) *reinterpret_cast<halfx8*>(buf + wdst[j]) = w.v[j];
     };
-    const int b_off = m * kRowW + 32 * g;
+    const int b_off = 16 * (tid & 63);
     auto compute = [&](const ARegs& a, const unsigned char* buf, float scale) {
         halfx8 ah[2], al[2];
 #pragma unroll
@@ -114,8 +114,8 @@ __device__ __forceinline__ void wfirst_gemm_tile(floatx16 (&acc)[kFNI], const _F
         for (int s = 0; s < 2; s++)
 #pragma unroll
             for (int ni = 0; ni < kFNI; ni++) {
-                const halfx8 bh = *reinterpret_cast<const halfx8*>(buf + b_off + ni * 32 * kRowW + 16 * s);
-                const halfx8 bl = *reinterpret_cast<const halfx8*>(buf + kPlaneW + b_off + ni * 32 * kRowW + 16 * s);
+                const halfx8 bh = *reinterpret_cast<const halfx8*>(buf + b_off + 2048 * ni + 1024 * s);
+                const halfx8 bl = *reinterpret_cast<const halfx8*>(buf + kPlaneW + b_off + 2048 * ni + 1024 * s);
                 // W first: D[i][j] with i the filter column in the block and j the edge
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bh, al[s], acc[ni], 0, 0, 0);
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bl, ah[s], acc[ni], 0, 0, 0);
@@ -183,7 +183,7 @@ painn_filter_message_kernel(const _Float16* __restrict__ Wp, const float* __rest
                             float* __restrict__ slots, long n_blocks, float* __restrict__ out_a,
                             float* __restrict__ out_v, int tiles_n, long tiles_total) {
     constexpr int kSlice = kFSlice, kRed = kFRed;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kFBufW];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kFLds];
     __shared__ __attribute__((aligned(16))) float wb[2 * kFTN];   // the tile's 1 / weight scale, then its bias
 
     const long bid = blockIdx.x;
@@ -376,7 +376,7 @@ linear_rowsum_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restr
                            float* __restrict__ Y, float* __restrict__ out, int tiles_n, long tiles_total,
                            float bound_mul, float bound_add) {
     constexpr int kSlice = kFSlice, kRed = kFRed;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kFBufW];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kFLds];
     __shared__ __attribute__((aligned(16))) float wb[2 * kFTN];   // the tile's 1 / weight scale, then its bias
 
     const long bid = blockIdx.x;
@@ -544,7 +544,7 @@ painn_filter_hidden_kernel(const _Float16* __restrict__ Wp, const float* __restr
                            const float* __restrict__ W1, long so, long si, const float* __restrict__ b1g, int hidden,
                            const float* __restrict__ h1_bound, float* __restrict__ Y, int tiles_n, long tiles_total) {
     constexpr int kSlice = kFSlice, kRed = kFRed;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kFBufW];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kFLds];
     __shared__ __attribute__((aligned(16))) float wb[2 * kFTN];
     __shared__ __attribute__((aligned(16))) _Float16 w1h[kHidMax * 16];
     __shared__ __attribute__((aligned(16))) _Float16 w1l[kHidMax * 16];

@@ -464,6 +464,72 @@ int launch_few_outputs(const float* W, long so, long si, const float* X, long R,
     return check_launch("mg_tensor_linear");
 }
 
+// A handful of input channels (one-hot atom types, the 8 radial functions, vector read-ins of one channel): the matrix
+// tiles above pad them to a multiple of 16 and write their output through LDS layouts made for long reductions, 70 us for
+// 65536 x 20 -> 256, where the output is written in 14.  Here a thread owns one output column (channel, component), keeps
+// its I weights in registers and walks over the rows of a tile, whose inputs are in LDS (the same word for all lanes when
+// T = 1).  Bound by the stores of y, which are unit stride in either layout.
+template <int T, int KMAX>
+__global__ void __launch_bounds__(256) linear_few_inputs_kernel(const float* __restrict__ W, long so, long si,
+                                                                const float* __restrict__ X, long R, int I, int O,
+                                                                const float* __restrict__ bias, int act, int accumulate,
+                                                                int y_comp_major, int tile_rows, float* __restrict__ Y) {
+    constexpr int kRow = KMAX * T;
+    __shared__ __attribute__((aligned(16))) float xs[64 * kRow];
+    const long r0 = (long)blockIdx.x * tile_rows;
+    const int rows = R - r0 < tile_rows ? (int)(R - r0) : tile_rows;
+    for (int k = threadIdx.x; k < rows * kRow; k += 256) {
+        const int r = k / kRow, c = k - r * kRow;
+        xs[k] = c < I * T ? X[(r0 + r) * (long)I * T + c] : 0.f;
+    }
+    const int Q = O * T;
+    const int q = (int)blockIdx.y * 256 + threadIdx.x;
+    const int o = q < Q ? (y_comp_major ? q % O : q / T) : 0;
+    const int t = q < Q ? (y_comp_major ? q / O : q % T) : 0;
+    float w[KMAX];
+#pragma unroll
+    for (int i = 0; i < KMAX; i++) w[i] = i < I ? W[(long)o * so + (long)i * si] : 0.f;
+    const float b = bias ? bias[o] : 0.f;
+    __syncthreads();
+    if (q >= Q) return;
+    float* y = Y + r0 * Q + q;
+    for (int r = 0; r < rows; r++) {
+        const float* x = xs + r * kRow + (T == 1 ? 0 : t);
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < KMAX; i++) sum = fmaf(w[i], x[i * T], sum);
+        float v = activate(sum + b, act);
+        if (accumulate) v += y[(long)r * Q];
+        y[(long)r * Q] = v;
+    }
+}
+
+constexpr int few_inputs_max(int T) { return T == 1 ? 32 : 8; }
+
+template <int T>
+int launch_few_inputs(const float* W, long so, long si, const float* X, long R, int I, int O, const float* bias, int act,
+                      int accumulate, int y_comp_major, float* Y, hipStream_t st) {
+    // tiles of 64 rows, fewer where that would leave CUs without work
+    const long cols = ceil_div((long)O * T, 256);
+    int tile = 64;
+    while (tile > 4 && ceil_div(R, tile) * cols < 512) tile >>= 1;
+    const long tiles = ceil_div(R, tile);
+    MG_REQUIRE(tiles <= 0x7fffffffL && cols <= 65535, "mg_tensor_linear: grid too large (rows=%ld dim_out=%d)", R, O);
+    const dim3 grid((unsigned)tiles, (unsigned)cols);
+#define MG_FEW(K)                                                                                                        \
+    hipLaunchKernelGGL((linear_few_inputs_kernel<T, K>), grid, dim3(256), 0, st, W, so, si, X, R, I, O, bias, act,       \
+                       accumulate, y_comp_major, tile, Y)
+    if (I <= 4) MG_FEW(4);
+    else if (I <= 8 || T > 1) MG_FEW(8);
+    else if constexpr (T == 1) {
+        if (I <= 16) MG_FEW(16);
+        else if (I <= 24) MG_FEW(24);
+        else MG_FEW(32);
+    }
+#undef MG_FEW
+    return check_launch("mg_tensor_linear");
+}
+
 }  // namespace
 }  // namespace mg
 
@@ -493,6 +559,12 @@ int mg_tensor_linear_layout(int inds, const float* W, long w_stride_o, long w_st
         if (inds == 0) return launch_few_outputs<1>(W, so, si, x, rows, dim_in, dim_out, b, act, accumulate, ycm, y, st);
         if (inds == 1) return launch_few_outputs<3>(W, so, si, x, rows, dim_in, dim_out, b, act, accumulate, ycm, y, st);
         return launch_few_outputs<9>(W, so, si, x, rows, dim_in, dim_out, b, act, accumulate, ycm, y, st);
+    }
+    if (dim_in >= 1 && dim_in <= few_inputs_max(T) && (x_layout == 0 || inds == 0)) {
+        const int ycm = (inds > 0 && y_layout == 1) ? 1 : 0;
+        if (inds == 0) return launch_few_inputs<1>(W, so, si, x, rows, dim_in, dim_out, b, act, accumulate, ycm, y, st);
+        if (inds == 1) return launch_few_inputs<3>(W, so, si, x, rows, dim_in, dim_out, b, act, accumulate, ycm, y, st);
+        return launch_few_inputs<9>(W, so, si, x, rows, dim_in, dim_out, b, act, accumulate, ycm, y, st);
     }
     if (inds == 0 || x_layout == 1) {
         // component-major input: every (row, comp) pair is an independent row of a plain GEMM

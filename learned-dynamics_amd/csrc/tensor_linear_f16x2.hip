@@ -20,8 +20,8 @@
 //     bytes, four 16-byte loads), two chunks ahead, and splits them in registers.  Every row is
 //     loaded and split exactly once per tile, nothing about x is tied to a barrier, and the LDS
 //     carries only W.
-//   * W planes (already fp16) go global -> registers -> LDS, double buffered, K chunk 32 (rows of
-//     64 B padded to 80 B: conflict free for 16-byte reads), one barrier per chunk.
+//   * W planes (already fp16, packed in fragment order: f16x2.hpp) go global -> registers -> LDS, double buffered, K
+//     chunk 32, one barrier per chunk.
 //   * the k order inside a chunk is a permutation (MFMA step s takes k = 16 g + 8 s .. + 8 from
 //     lane group g); W is read from LDS with the same permutation, so the products pair up.
 //   * loads are never predicated (rows past the end are clamped to the last row, whose
@@ -54,26 +54,73 @@ __device__ __forceinline__ float activate_c(float v) {
     return v;
 }
 
-// one wave per output row: row maximum -> scale -> hi / lo planes (O_pad rows, zero filled) + 1/scale per row
-__global__ void __launch_bounds__(256) pack_weight_f16x2_kernel(const float* __restrict__ W, long so, long si, int I,
-                                                                int O, int O_pad, _Float16* __restrict__ planes,
-                                                                float* __restrict__ inv_scale) {
-    const int lane = threadIdx.x & 63;
+// Weight planes in fragment order (f16x2.hpp) + 1/scale per row: a workgroup takes a block of 32 output rows (rows past O
+// are zeros), a thread pieces of 8 k of one row, kept in registers between the row maximum (LDS, max of the bit patterns
+// of |w|: any order gives the same) and the split.  One pass over W for I <= kPackRegs * 256.  I_w <= I: columns of W, the
+// others are zeros.
+constexpr int kPackThreads = 1024, kPackRegs = 4;
+__global__ void __launch_bounds__(kPackThreads) pack_weight_f16x2_kernel(const float* __restrict__ W, long so, long si, int I_w,
+                                                                         int I, int O, int O_pad, _Float16* __restrict__ planes,
+                                                                         float* __restrict__ inv_scale) {
+    __shared__ unsigned row_max[32];
+    const int tid = threadIdx.x;
+    const int block = blockIdx.x;
+    const int m = tid & 31;
+    const long o = 32L * block + m;
+    const int pieces = I >> 3;                            // per row; thread t takes pieces t / 32, + 32, ...
     const long total = (long)O_pad * I;
-    for (long o = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6; o < O_pad; o += ((long)gridDim.x * blockDim.x) >> 6) {
-        float amax = 0.f;
-        if (o < O)
-            for (int i = lane; i < I; i += 64) amax = fmaxf(amax, fabsf(W[o * so + (long)i * si]));
-        for (int d = 1; d < 64; d <<= 1) amax = fmaxf(amax, __shfl_xor(amax, d));
-        float inv;
-        const float s = pow2_scale(amax, &inv);
-        for (int i = lane; i < I; i += 64) {
-            const float v = o < O ? W[o * so + (long)i * si] * s : 0.f;
-            const _Float16 h = (_Float16)v;
-            planes[o * I + i] = h;
-            planes[total + o * I + i] = (_Float16)(v - (float)h);
+    if (tid < 32) row_max[tid] = 0;
+    __syncthreads();
+    const float* row = W + (o < O ? o : 0) * so;
+    auto load = [&](float (&v)[8], int piece) {
+        const float* p = row + (long)(8 * piece) * si;
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = o < O && 8 * piece + j < I_w ? p[j * si] : 0.f;
+    };
+    float keep[kPackRegs][8];
+    unsigned mx = 0;
+#pragma unroll
+    for (int u = 0; u < kPackRegs; u++) {
+        const int piece = (tid >> 5) + 32 * u;
+        if (piece < pieces) {
+            load(keep[u], piece);
+#pragma unroll
+            for (int j = 0; j < 8; j++) { const unsigned b = __float_as_uint(fabsf(keep[u][j])); mx = b > mx ? b : mx; }
         }
-        if (lane == 0) inv_scale[o] = inv;
+    }
+    for (int piece = (tid >> 5) + 32 * kPackRegs; piece < pieces; piece += 32) {
+        float v[8];
+        load(v, piece);
+#pragma unroll
+        for (int j = 0; j < 8; j++) { const unsigned b = __float_as_uint(fabsf(v[j])); mx = b > mx ? b : mx; }
+    }
+    atomicMax(&row_max[m], mx);
+    __syncthreads();
+    float inv;
+    const float s = pow2_scale(__uint_as_float(row_max[m]), &inv);
+    if (tid < 32) inv_scale[o] = inv;
+    auto store = [&](const float (&v)[8], int piece) {
+        halfx8 hi, lo;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const float x = v[j] * s;
+            const _Float16 h = (_Float16)x;
+            hi[j] = h;
+            lo[j] = (_Float16)(x - (float)h);
+        }
+        const long at = packed_index(o, 8 * piece, I);
+        *reinterpret_cast<halfx8*>(planes + at) = hi;
+        *reinterpret_cast<halfx8*>(planes + total + at) = lo;
+    };
+#pragma unroll
+    for (int u = 0; u < kPackRegs; u++) {
+        const int piece = (tid >> 5) + 32 * u;
+        if (piece < pieces) store(keep[u], piece);
+    }
+    for (int piece = (tid >> 5) + 32 * kPackRegs; piece < pieces; piece += 32) {
+        float v[8];
+        load(v, piece);
+        store(v, piece);
     }
 }
 
@@ -128,9 +175,9 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
                          const float* __restrict__ xmax, int xmax_parts, long xmax_stride, long xmax_div, long R, int I,
                          int O, int O_pad, const float* __restrict__ bias, int act, int accumulate,
                          float* __restrict__ Y, float* __restrict__ ymax, int tiles_n, long tiles_total, int out_T,
-                         float bound_mul, float bound_add) {
+                         float bound_mul, float bound_add, long bias_rows) {
     constexpr int TM = 32 * WAVES, TN = 32 * NI, THREADS = 64 * WAVES;
-    constexpr int kPlaneW = TN * kRowW, kBufW = 2 * kPlaneW;
+    constexpr int kPlaneW = TN * 64, kBufW = 2 * kPlaneW;
     constexpr int kPieces = 8 * TN;                          // 16-byte pieces of W per chunk (2 planes x TN rows x 4)
     constexpr int kPer = (kPieces + THREADS - 1) / THREADS;  // per thread
     __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kBufW];
@@ -176,9 +223,9 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
     for (int j = 0; j < kPer; j++) {
         int q = tid + THREADS * j;
         if (q >= kPieces) q = kPieces - 1;                    // surplus threads repeat the last piece
-        const int plane = q / (4 * TN), row = (q % (4 * TN)) >> 2, piece = q & 3;
-        wsrc[j] = Wp + plane * plane_elems + (long)(n0 + row) * I + 8 * piece;
-        wdst[j] = plane * kPlaneW + row * kRowW + piece * 16;
+        const int plane = q / (4 * TN), i = q % (4 * TN);
+        wsrc[j] = Wp + plane * plane_elems + packed_piece(n0, i, I);
+        wdst[j] = plane * kPlaneW + 16 * i;
     }
     const int k_last = I - kCK;
 
@@ -192,13 +239,13 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
     auto load_w = [&](WRegs& w, int k0) {
         k0 = k0 < I ? k0 : k_last;
 #pragma unroll
-        for (int j = 0; j < kPer; j++) w.v[j] = *reinterpret_cast<const halfx8*>(wsrc[j] + k0);
+        for (int j = 0; j < kPer; j++) w.v[j] = *reinterpret_cast<const halfx8*>(wsrc[j] + 32L * k0);
     };
     auto store_w = [&](const WRegs& w, unsigned char* buf) {
 #pragma unroll
         for (int j = 0; j < kPer; j++) *reinterpret_cast<halfx8*>(buf + wdst[j]) = w.v[j];
     };
-    const int b_off = m * kRowW + 32 * g;
+    const int b_off = 16 * lane;
     auto compute = [&](const ARegs& a, const unsigned char* buf, float scale) {
         halfx8 ah[2], al[2];
 #pragma unroll
@@ -214,8 +261,8 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
         for (int s = 0; s < 2; s++)
 #pragma unroll
             for (int ni = 0; ni < NI; ni++) {
-                const halfx8 bh = *reinterpret_cast<const halfx8*>(buf + b_off + ni * 32 * kRowW + 16 * s);
-                const halfx8 bl = *reinterpret_cast<const halfx8*>(buf + kPlaneW + b_off + ni * 32 * kRowW + 16 * s);
+                const halfx8 bh = *reinterpret_cast<const halfx8*>(buf + b_off + 2048 * ni + 1024 * s);
+                const halfx8 bl = *reinterpret_cast<const halfx8*>(buf + kPlaneW + b_off + 2048 * ni + 1024 * s);
                 // small terms first
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[s], bh, acc[ni], 0, 0, 0);
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s], bl, acc[ni], 0, 0, 0);
@@ -255,9 +302,10 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
 
     const bool full_cols = n0 + TN <= O;
     // ---- fast path, plain rows: y (rows, O)
-    auto epilogue_rows = [&](auto act_tag, auto acc_tag) {
+    auto epilogue_rows = [&](auto act_tag, auto acc_tag, auto some_tag) {
         constexpr int kAct = decltype(act_tag)::value;
         constexpr bool kAccumulate = decltype(acc_tag)::value;
+        constexpr bool kSomeBias = decltype(some_tag)::value;      // only rows below bias_rows have the bias
         float bv[NI], iw[NI];
 #pragma unroll
         for (int ni = 0; ni < NI; ni++) {
@@ -274,7 +322,8 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
                 float mx = 0.f;
 #pragma unroll
                 for (int ni = 0; ni < NI; ni++) {
-                    float v = activate_c<kAct>(acc[ni][q] * isx * iw[ni] + bv[ni]);
+                    const float b = kSomeBias && r >= bias_rows ? 0.f : bv[ni];
+                    float v = activate_c<kAct>(acc[ni][q] * isx * iw[ni] + b);
                     if constexpr (kAccumulate) v += yrow[ni * 32];
                     yrow[ni * 32] = v;
                     mx = fmaxf(mx, fabsf(v));
@@ -311,14 +360,18 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
         }
     };
     if (full_cols && out_T == 1) {
-        if (accumulate) {
-            if (act == 1) epilogue_rows(std::integral_constant<int, 1>{}, std::true_type{});
-            else if (act == 2) epilogue_rows(std::integral_constant<int, 2>{}, std::true_type{});
-            else epilogue_rows(std::integral_constant<int, 0>{}, std::true_type{});
+        constexpr std::integral_constant<int, 0> kNone{};
+        constexpr std::integral_constant<int, 1> kSilu{};
+        constexpr std::integral_constant<int, 2> kLeaky{};
+        if (bias_rows < R) epilogue_rows(kNone, std::false_type{}, std::true_type{});   // (no activation, not accumulated)
+        else if (accumulate) {
+            if (act == 1) epilogue_rows(kSilu, std::true_type{}, std::false_type{});
+            else if (act == 2) epilogue_rows(kLeaky, std::true_type{}, std::false_type{});
+            else epilogue_rows(kNone, std::true_type{}, std::false_type{});
         } else {
-            if (act == 1) epilogue_rows(std::integral_constant<int, 1>{}, std::false_type{});
-            else if (act == 2) epilogue_rows(std::integral_constant<int, 2>{}, std::false_type{});
-            else epilogue_rows(std::integral_constant<int, 0>{}, std::false_type{});
+            if (act == 1) epilogue_rows(kSilu, std::false_type{}, std::false_type{});
+            else if (act == 2) epilogue_rows(kLeaky, std::false_type{}, std::false_type{});
+            else epilogue_rows(kNone, std::false_type{}, std::false_type{});
         }
         return;
     }
@@ -342,7 +395,7 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
             if (r < R) {
                 const long row = r / out_T;
                 const long addr = (row * O + n) * out_T + (r - row * out_T);
-                float v = activate(acc[ni][q] * inv_sx[rl] * iw + bv, act);
+                float v = activate(acc[ni][q] * inv_sx[rl] * iw + (r < bias_rows ? bv : 0.f), act);
                 if (accumulate) v += Y[addr];
                 Y[addr] = v;
                 rmax[q] = fmaxf(rmax[q], fabsf(v));
@@ -373,7 +426,8 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
                                 const float* __restrict__ X, const float* __restrict__ xmax, int xmax_parts,
                                 long xmax_stride, long xmax_div, long R, int I, int O, int O_pad,
                                 const float* __restrict__ bias, int act, int accumulate, float* __restrict__ Y,
-                                float* __restrict__ ymax, int tiles_n, int out_T, float bound_mul, float bound_add) {
+                                float* __restrict__ ymax, int tiles_n, int out_T, float bound_mul, float bound_add,
+                                long bias_rows) {
     constexpr int TN = 32 * NI, THREADS = 64 * WAVES;
     constexpr int kPitch = TN + 1;                            // floats per row of a partial tile
     __shared__ float partial[WAVES][32 * kPitch];
@@ -402,7 +456,7 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
         if (wave == 0 && g == 0) inv_sx[m] = inv;
     }
     // lane's fragment of W for MFMA step s, column block ni: row n0 + 32 ni + m, k = k0 + 16 g + 8 s .. + 8
-    const _Float16* wrow = Wp + (long)(n0 + m) * I + 16 * g;
+    const _Float16* wrow = Wp + packed_piece(n0, lane, I);
 
     floatx16 acc[NI];
 #pragma unroll
@@ -419,8 +473,8 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
         for (int ni = 0; ni < NI; ni++)
 #pragma unroll
             for (int s2 = 0; s2 < 2; s2++) {
-                c.wh[ni][s2] = *reinterpret_cast<const halfx8*>(wrow + (long)ni * 32 * I + k0 + 8 * s2);
-                c.wl[ni][s2] = *reinterpret_cast<const halfx8*>(wrow + plane_elems + (long)ni * 32 * I + k0 + 8 * s2);
+                c.wh[ni][s2] = *reinterpret_cast<const halfx8*>(wrow + (long)ni * 32 * I + 32L * k0 + 512 * s2);
+                c.wl[ni][s2] = *reinterpret_cast<const halfx8*>(wrow + plane_elems + (long)ni * 32 * I + 32L * k0 + 512 * s2);
             }
 #pragma unroll
         for (int j = 0; j < 4; j++) c.a[j] = *reinterpret_cast<const float4*>(xrow + k0 + 4 * j);
@@ -463,7 +517,7 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
     // a thread finishes the elements e = tid, tid + THREADS, ...: row e / TN, column e % TN (the TN / 1 lanes of a
     // row are neighbours, so its maximum is a shuffle away)
     constexpr int kPer = 32 * TN / THREADS;
-    static_assert(32 * TN % THREADS == 0 && THREADS % TN == 0, "whole rows per pass");
+    static_assert(32 * TN % THREADS == 0 && THREADS % TN == 0 && TN <= 64, "whole rows per pass, a row within a wave");
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
         const int e = tid + THREADS * j;
@@ -477,7 +531,7 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
         if (r < R && n < O) {
             const long row = r / out_T;
             const long addr = (row * O + n) * out_T + (r - row * out_T);
-            v = activate(sum * inv_sx[rl] * w_inv[n] + (bias ? bias[n] : 0.f), act);
+            v = activate(sum * inv_sx[rl] * w_inv[n] + (bias && r < bias_rows ? bias[n] : 0.f), act);
             if (accumulate) v += Y[addr];
             Y[addr] = v;
         }
@@ -492,14 +546,24 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
 
 inline int o_pad_of(int dim_out) { return (dim_out + 255) / 256 * 256; }
 
-// the split-K kernel's domain: one column tile of at most 64 columns (the packed planes are zero filled up to a
-// multiple of 256 rows, so a partly used tile reads zeros), at least 16 chunks of K, and few rows.  Measured
-// against the row-streaming kernel for K = 512 .. 2048: 11 - 19 us against 13 - 67 us up to 6144 rows; from
-// about 12 000 rows on the row-streaming kernel (which reads W once per 256 rows and keeps more of x in flight)
-// is level or ahead, except at 16 columns or fewer, where its 32-column tile is half empty (31 against 48 us at
-// 18 432 rows, K = 1280).
-inline bool use_splitk(long R, int I, int O) {
-    return O <= 64 && I >= 512 && (R <= 8192 || (O <= 16 && R <= 32768));
+// The split-K kernel is for problems whose row-streaming tiles would leave most of the chip idle while a few workgroups walk
+// K one barrier at a time.  The rule is the measured crossover (R = 337 .. 49152, K = 128 .. 1280, O = 64 .. 512) in units
+// of 32 x 32 output blocks:
+//   up to 256 blocks      one block per workgroup, eight waves on K     512 -> 512 at 337 rows  5.3 us (streaming 12.7)
+//   up to 512 blocks      two column blocks per workgroup               512 -> 512 at 1024 rows 7.4 us (13.4)
+//   up to 1536 blocks     two column blocks, four waves on K            512 -> 512 at 3072 rows 16.8 us (22.1)
+//   more                  row streaming (W read once per 128 or 256 rows): 512 -> 512 at 4096 rows 22.5 us (23.0 split)
+// K below 256 has fewer than eight chunks: four waves.  At most 64 column tiles (row maxima per tile).
+struct SplitK {
+    int waves, ni;       // waves = 0: the row-streaming kernel
+};
+inline SplitK choose_splitk(long R, int I, int O) {
+    const long blocks = ceil_div(R, 32) * ceil_div(O, 32);
+    if (blocks > 1536 || O > 2048) return SplitK{0, 0};
+    if (I < 256) return SplitK{4, blocks <= 896 || O <= 32 ? 1 : 2};
+    if (O <= 32) return SplitK{8, 1};
+    if (blocks <= 256) return SplitK{8, 1};
+    return SplitK{blocks <= 512 ? 8 : 4, 2};
 }
 
 struct Shape {
@@ -538,7 +602,7 @@ inline Shape choose_shape(long R, int I, int O) {
 template <int WAVES, int NI>
 int launch(const _Float16* planes, const float* w_inv, const float* x, const float* xmax, int parts, long stride,
            long div, long rows, int I, int O, int O_pad, const float* bias, int act, int accumulate, float* y,
-           float* ymax, int out_T, float bound_mul, float bound_add, hipStream_t st) {
+           float* ymax, int out_T, float bound_mul, float bound_add, long bias_rows, hipStream_t st) {
     const long tiles_m = ceil_div(rows, 32 * WAVES);
     const int tiles_n = (int)ceil_div(O, 32 * NI);
     const long total = tiles_m * tiles_n;
@@ -546,7 +610,7 @@ int launch(const _Float16* planes, const float* w_inv, const float* x, const flo
     MG_REQUIRE(grid <= 0x7fffffffL, "mg_tensor_linear_f16x2: grid too large (rows=%ld dim_out=%d)", rows, O);
     hipLaunchKernelGGL((linear_rows_f16x2_kernel<WAVES, NI>), dim3((unsigned)grid), dim3(64 * WAVES), 0, st, planes,
                        w_inv, x, xmax, parts, stride, div, rows, I, O, O_pad, bias, act, accumulate, y, ymax, tiles_n,
-                       total, out_T, bound_mul, bound_add);
+                       total, out_T, bound_mul, bound_add, bias_rows);
     return check_launch("mg_tensor_linear_f16x2");
 }
 
@@ -564,18 +628,23 @@ int mg_linear_f16x2_packed_weight_bytes(int dim_in, int dim_out, size_t* bytes) 
     return MG_OK;
 }
 
-int mg_linear_f16x2_pack_weight(const float* W, long w_stride_o, long w_stride_i, int dim_in, int dim_out,
-                                void* packed, mg_stream_t stream) {
-    MG_REQUIRE(dim_in >= 0 && dim_out >= 0, "mg_linear_f16x2_pack_weight: negative size");
+int mg_linear_f16x2_pack_weight_padded(const float* W, long w_stride_o, long w_stride_i, int dim_in, int dim_out, int dim_pad,
+                                       void* packed, mg_stream_t stream) {
+    MG_REQUIRE(dim_in >= 0 && dim_out >= 0 && dim_pad >= dim_in, "mg_linear_f16x2_pack_weight: bad size");
     if (dim_in == 0 || dim_out == 0) return MG_OK;
     MG_REQUIRE(W && packed && aligned16(packed), "mg_linear_f16x2_pack_weight: null or unaligned pointer");
-    MG_REQUIRE(dim_in % 8 == 0, "mg_linear_f16x2_pack_weight: dim_in must be a multiple of 8");
+    MG_REQUIRE(dim_pad % 32 == 0, "mg_linear_f16x2_pack_weight: dim_in must be a multiple of 32");
     const int O_pad = o_pad_of(dim_out);
     _Float16* planes = static_cast<_Float16*>(packed);
-    float* inv = reinterpret_cast<float*>(planes + 2L * O_pad * dim_in);
-    hipLaunchKernelGGL(pack_weight_f16x2_kernel, dim3((unsigned)ceil_div(O_pad, 4)), dim3(256), 0, (hipStream_t)stream,
-                       W, w_stride_o, w_stride_i, dim_in, dim_out, O_pad, planes, inv);
+    float* inv = reinterpret_cast<float*>(planes + 2L * O_pad * dim_pad);
+    hipLaunchKernelGGL(pack_weight_f16x2_kernel, dim3((unsigned)(O_pad / 32)), dim3(kPackThreads), 0, (hipStream_t)stream,
+                       W, w_stride_o, w_stride_i, dim_in, dim_pad, dim_out, O_pad, planes, inv);
     return check_launch("mg_linear_f16x2_pack_weight");
+}
+
+int mg_linear_f16x2_pack_weight(const float* W, long w_stride_o, long w_stride_i, int dim_in, int dim_out,
+                                void* packed, mg_stream_t stream) {
+    return mg_linear_f16x2_pack_weight_padded(W, w_stride_o, w_stride_i, dim_in, dim_out, dim_in, packed, stream);
 }
 
 int mg_row_absmax(const float* x, long rows, int dim, float* out, mg_stream_t stream) {
@@ -602,9 +671,18 @@ int mg_components_to_rows(const float* x, long rows, int dim, int comps, int dim
     return check_launch("mg_components_to_rows");
 }
 
-int mg_tensor_linear_f16x2_rowmax_parts(long rows, int dim_in, int dim_out) {
-    if (use_splitk(rows, dim_in, dim_out)) return 1;
+int mg_tensor_linear_f16x2_rowmax_parts_sequential(long rows, int dim_in, int dim_out) {
     return (int)ceil_div(dim_out, 32 * choose_shape(rows, dim_in, dim_out).ni);
+}
+
+int mg_tensor_linear_f16x2_rowmax_parts(long rows, int dim_in, int dim_out) {
+    const SplitK sk = choose_splitk(rows, dim_in, dim_out);
+    if (sk.waves) return (int)ceil_div(dim_out, 32 * sk.ni);
+    return (int)ceil_div(dim_out, 32 * choose_shape(rows, dim_in, dim_out).ni);
+}
+
+int mg_tensor_linear_f16x2_splits_k(long rows, int dim_in, int dim_out) {
+    return choose_splitk(rows, dim_in, dim_out).waves != 0;
 }
 
 int mg_tensor_linear_f16x2(const void* packed_W, const float* x, const float* x_rowmax, int x_rowmax_parts,
@@ -620,41 +698,58 @@ int mg_tensor_linear_f16x2_scaled_bound(const void* packed_W, const float* x, co
                                         long x_rowmax_stride, long x_rows_per_bound, long rows, int dim_in, int dim_out,
                                         const float* bias, int act, int accumulate, int out_comps, float* y,
                                         float* y_rowmax, float bound_mul, float bound_add, mg_stream_t stream) {
-    MG_REQUIRE(bound_mul >= 0.f && bound_add >= 0.f && bound_mul == bound_mul && bound_add == bound_add,
+    const mg_f16x2_linear a{packed_W,  x,    x_rowmax, x_rowmax_parts, x_rowmax_stride, x_rows_per_bound, bound_mul, bound_add,
+                            rows,      dim_in, dim_out, bias,          rows,            act,              accumulate, out_comps,
+                            0,         y,    y_rowmax};
+    return mg_tensor_linear_f16x2_run(&a, stream);
+}
+
+int mg_tensor_linear_f16x2_run(const mg_f16x2_linear* args, mg_stream_t stream) {
+    MG_REQUIRE(args != nullptr, "mg_tensor_linear_f16x2: null pointer");
+    const mg_f16x2_linear& a = *args;
+    MG_REQUIRE(a.bound_mul >= 0.f && a.bound_add >= 0.f && a.bound_mul == a.bound_mul && a.bound_add == a.bound_add,
                "mg_tensor_linear_f16x2: the bound's factor and offset must be non-negative numbers");
-    MG_REQUIRE(rows >= 0 && dim_in > 0 && dim_out >= 0, "mg_tensor_linear_f16x2: bad size");
-    MG_REQUIRE(dim_in % 32 == 0, "mg_tensor_linear_f16x2: dim_in must be a multiple of 32");
-    MG_REQUIRE(act >= 0 && act <= 2, "mg_tensor_linear_f16x2: unknown activation %d", act);
-    MG_REQUIRE(out_comps == 1 || out_comps == 3 || out_comps == 9, "mg_tensor_linear_f16x2: out_comps must be 1, 3 or 9");
-    MG_REQUIRE(x_rowmax_parts >= 1 && x_rowmax_parts <= 64, "mg_tensor_linear_f16x2: x_rowmax_parts must be in 1..64");
-    MG_REQUIRE(x_rowmax_stride == 0 || x_rowmax_stride >= x_rowmax_parts,
+    MG_REQUIRE(a.rows >= 0 && a.dim_in > 0 && a.dim_out >= 0, "mg_tensor_linear_f16x2: bad size");
+    MG_REQUIRE(a.dim_in % 32 == 0, "mg_tensor_linear_f16x2: dim_in must be a multiple of 32");
+    MG_REQUIRE(a.act >= 0 && a.act <= 2, "mg_tensor_linear_f16x2: unknown activation %d", a.act);
+    MG_REQUIRE(a.out_comps == 1 || a.out_comps == 3 || a.out_comps == 9, "mg_tensor_linear_f16x2: out_comps must be 1, 3 or 9");
+    MG_REQUIRE(a.x_rowmax_parts >= 1 && a.x_rowmax_parts <= 64, "mg_tensor_linear_f16x2: x_rowmax_parts must be in 1..64");
+    MG_REQUIRE(a.x_rowmax_stride == 0 || a.x_rowmax_stride >= a.x_rowmax_parts,
                "mg_tensor_linear_f16x2: x_rowmax_stride must be 0 (one bound for all rows) or >= x_rowmax_parts");
-    MG_REQUIRE(x_rows_per_bound >= 1, "mg_tensor_linear_f16x2: x_rows_per_bound must be positive");
-    MG_REQUIRE(y_rowmax == nullptr || out_comps == 1, "mg_tensor_linear_f16x2: y_rowmax needs out_comps == 1");
-    if (rows == 0 || dim_out == 0) return MG_OK;
-    MG_REQUIRE(packed_W && x && y && x_rowmax && aligned16(x) && aligned16(packed_W),
+    MG_REQUIRE(a.x_rows_per_bound >= 1, "mg_tensor_linear_f16x2: x_rows_per_bound must be positive");
+    MG_REQUIRE(a.y_rowmax == nullptr || a.out_comps == 1, "mg_tensor_linear_f16x2: y_rowmax needs out_comps == 1");
+    MG_REQUIRE(a.bias_rows >= a.rows || (a.bias_rows >= 0 && a.act == 0 && !a.accumulate && a.out_comps == 1),
+               "mg_tensor_linear_f16x2: a bias for some rows only goes with plain rows, no activation, not accumulated");
+    if (a.rows == 0 || a.dim_out == 0) return MG_OK;
+    MG_REQUIRE(a.packed_W && a.x && a.y && a.x_rowmax && aligned16(a.x) && aligned16(a.packed_W),
                "mg_tensor_linear_f16x2: null or unaligned pointer");
-    const int O_pad = o_pad_of(dim_out);
-    const _Float16* planes = static_cast<const _Float16*>(packed_W);
-    const float* w_inv = reinterpret_cast<const float*>(planes + 2L * O_pad * dim_in);
+    const int O_pad = o_pad_of(a.dim_out);
+    const _Float16* planes = static_cast<const _Float16*>(a.packed_W);
+    const float* w_inv = reinterpret_cast<const float*>(planes + 2L * O_pad * a.dim_in);
     hipStream_t st = (hipStream_t)stream;
-    if (use_splitk(rows, dim_in, dim_out)) {
-        const long tiles = ceil_div(rows, 32);
-        MG_REQUIRE(tiles <= 0x7fffffffL, "mg_tensor_linear_f16x2: grid too large (rows=%ld)", rows);
-        if (dim_out <= 32)
-            hipLaunchKernelGGL((linear_rows_splitk_f16x2_kernel<8, 1>), dim3((unsigned)tiles), dim3(512), 0, st, planes,
-                               w_inv, x, x_rowmax, x_rowmax_parts, x_rowmax_stride, x_rows_per_bound, rows, dim_in,
-                               dim_out, O_pad, bias, act, accumulate, y, y_rowmax, 1, out_comps, bound_mul, bound_add);
-        else
-            hipLaunchKernelGGL((linear_rows_splitk_f16x2_kernel<8, 2>), dim3((unsigned)tiles), dim3(512), 0, st, planes,
-                               w_inv, x, x_rowmax, x_rowmax_parts, x_rowmax_stride, x_rows_per_bound, rows, dim_in,
-                               dim_out, O_pad, bias, act, accumulate, y, y_rowmax, 1, out_comps, bound_mul, bound_add);
+    const SplitK sk = a.sequential ? SplitK{0, 0} : choose_splitk(a.rows, a.dim_in, a.dim_out);
+    if (sk.waves) {
+        const int tiles_n = (int)ceil_div(a.dim_out, 32 * sk.ni);
+        const long tiles = ceil_div(a.rows, 32) * tiles_n;
+        MG_REQUIRE(tiles <= 0x7fffffffL, "mg_tensor_linear_f16x2: grid too large (rows=%ld)", a.rows);
+#define MG_SPLITK(WV, N)                                                                                                   \
+    if (sk.waves == WV && sk.ni == N)                                                                                      \
+        hipLaunchKernelGGL((linear_rows_splitk_f16x2_kernel<WV, N>), dim3((unsigned)tiles), dim3(64 * WV), 0, st, planes,  \
+                           w_inv, a.x, a.x_rowmax, a.x_rowmax_parts, a.x_rowmax_stride, a.x_rows_per_bound, a.rows,        \
+                           a.dim_in, a.dim_out, O_pad, a.bias, a.act, a.accumulate, a.y, a.y_rowmax, tiles_n, a.out_comps, \
+                           a.bound_mul, a.bound_add, a.bias_rows)
+        MG_SPLITK(8, 1);
+        MG_SPLITK(8, 2);
+        MG_SPLITK(4, 1);
+        MG_SPLITK(4, 2);
+#undef MG_SPLITK
         return check_launch("mg_tensor_linear_f16x2");
     }
-    const Shape sh = choose_shape(rows, dim_in, dim_out);
-#define MG_F16X2_LAUNCH(WV, N)                                                                                       \
-    return launch<WV, N>(planes, w_inv, x, x_rowmax, x_rowmax_parts, x_rowmax_stride, x_rows_per_bound, rows, dim_in, \
-                         dim_out, O_pad, bias, act, accumulate, y, y_rowmax, out_comps, bound_mul, bound_add, st)
+    const Shape sh = choose_shape(a.rows, a.dim_in, a.dim_out);
+#define MG_F16X2_LAUNCH(WV, N)                                                                                             \
+    return launch<WV, N>(planes, w_inv, a.x, a.x_rowmax, a.x_rowmax_parts, a.x_rowmax_stride, a.x_rows_per_bound, a.rows,  \
+                         a.dim_in, a.dim_out, O_pad, a.bias, a.act, a.accumulate, a.y, a.y_rowmax, a.out_comps,            \
+                         a.bound_mul, a.bound_add, a.bias_rows, st)
     if (sh.waves == 8) {
         if (sh.ni == 1) MG_F16X2_LAUNCH(8, 1);
         if (sh.ni == 2) MG_F16X2_LAUNCH(8, 2);
