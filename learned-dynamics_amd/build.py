@@ -1,5 +1,5 @@
 """Build libmanagan_hip.so (the C-ABI library) for gfx950 with hipcc, and managan_torch_ext.so, the
-thin PyTorch C++ binding of it (host code only: csrc/torch_binding.cpp, compiled with g++ against
+thin PyTorch C++ binding of it (host code only: csrc/torch_binding.cpp and torch_ops.cpp, compiled with g++ against
 torch's headers and linked to the library next to it).
 
 Run as `python learned-dynamics_amd/build.py` or call build().  hipcc
@@ -72,18 +72,28 @@ def build_torch_binding():
 
     import torch
     tdir = os.path.dirname(torch.__file__)
-    cmd = ["g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-Wall", "-Wno-unused-function",
-           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=managan_torch_ext",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           "-I", INCLUDE, "-I", os.path.join(tdir, "include"),
-           "-I", os.path.join(tdir, "include", "torch", "csrc", "api", "include"), "-I", "/opt/rocm/include",
-           "-I", sysconfig.get_paths()["include"],
-           os.path.join(CSRC, "torch_binding.cpp"), "-o", EXT,
-           "-L", os.path.join(tdir, "lib"), "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip", "-ltorch_hip",
-           "-L", HERE, "-l:libmanagan_hip.so", "-Wl,-rpath,$ORIGIN"]
+    flags = ["-O2", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
+             "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=managan_torch_ext",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+             "-I", INCLUDE, "-I", os.path.join(tdir, "include"),
+             "-I", os.path.join(tdir, "include", "torch", "csrc", "api", "include"), "-I", "/opt/rocm/include",
+             "-I", sysconfig.get_paths()["include"]]
+
+    def compile_cpp(src):
+        os.makedirs(os.path.join(CSRC, "_obj"), exist_ok=True)
+        obj = os.path.join(CSRC, "_obj", src.replace(".cpp", "_cpp.o"))
+        r = subprocess.run(["g++", "-c", os.path.join(CSRC, src), "-o", obj] + flags, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"g++ failed on {src}:\n{r.stdout}\n{r.stderr}")
+        return obj
+    with ThreadPoolExecutor(max_workers=2) as ex:
+        objs = list(ex.map(compile_cpp, ("torch_binding.cpp", "torch_ops.cpp")))
+    cmd = ["g++", "-shared", "-o", EXT] + objs + [
+        "-L", os.path.join(tdir, "lib"), "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip", "-ltorch_hip",
+        "-L", HERE, "-l:libmanagan_hip.so", "-Wl,-rpath,$ORIGIN"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
-        raise RuntimeError(f"g++ failed on torch_binding.cpp:\n{r.stdout}\n{r.stderr}")
+        raise RuntimeError(f"linking managan_torch_ext.so failed:\n{r.stdout}\n{r.stderr}")
     return EXT
 
 

@@ -5,14 +5,12 @@
 //   tensor_ops_cuda       tensor_linear, differentiable (extensions/tensor_ops/tensor_ops.cpp:31-182)
 //   codegen_tensops_cuda  bee_fwd / bee_bwl / bee_bwr, cow_o0 / cow_o1 fwd / bwl / bwr
 //                         (extensions/codegen_tensops/codegen_tensops.cpp:1519-1978)
+// and of the radius graph and TensorProds; torch_ops.cpp holds the linears and the PaiNN layers.
 // Every function validates like the reference's front end (same messages), allocates its outputs with torch on the
 // inputs' device, and enqueues on torch's current stream of that device.  No arithmetic happens here: the kernels are
 // in libmanagan_hip.so.  Host C++ only (compiled with the host compiler: no device code, no GPU runtime calls of its
 // own), so that a call costs a few microseconds of host time where the ctypes route costs about twelve.
-#include <torch/extension.h>
-// torch's ROCm build presents its devices under the device type "cuda": the guard and stream types that know this
-#include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
-#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include "torch_common.hpp"
 
 #include <algorithm>
 #include <array>
@@ -21,38 +19,14 @@
 #include <cstdint>
 #include <map>
 #include <mutex>
-#include <string>
 #include <tuple>
-#include <vector>
 
-#include "managan_hip.h"
+using namespace mgt;
 
 namespace {
 
 constexpr const char* kBeeOrder[13] = {"000", "110", "220", "011", "101", "121", "211",
                                        "022", "202", "112", "222", "111", "212"};
-
-void check_input(const at::Tensor& t, const char* name, at::ScalarType dtype = at::kFloat) {
-    TORCH_CHECK(t.is_cuda(), name, " must be a CUDA tensor");
-    TORCH_CHECK(t.is_contiguous(), name, " must be contiguous");
-    TORCH_CHECK(t.scalar_type() == dtype, "expected scalar type ", c10::toString(dtype), " but found ",
-                c10::toString(t.scalar_type()), " for ", name);
-}
-
-// a non-zero status as the exception the reference would raise (the same texts as the ctypes route)
-void check(int status) {
-    if (status == MG_OK) return;
-    TORCH_CHECK(status != MG_ERR_BOX_TOO_SMALL, "box dimension must be greater than 3*cutoff");
-    const char* text = mg_last_error();
-    TORCH_CHECK(false, mg_status_string(status), text[0] ? ": " : "", text);
-}
-
-mg_stream_t stream_of(const at::Tensor& t) {
-    return reinterpret_cast<mg_stream_t>(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream());
-}
-
-const float* fp(const at::Tensor& t) { return t.data_ptr<float>(); }
-float* fp(at::Tensor& t) { return t.data_ptr<float>(); }
 
 std::vector<int64_t> shape_of(int64_t rows, int64_t chan, int rank) {
     std::vector<int64_t> s{rows, chan};
@@ -538,6 +512,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     // TensorProds.forward (managan/tensor_products.py:109-121) as one launch
     m.def("tensor_prods_supported", &tensor_prods_supported);
     m.def("tensor_prods", &tensor_prods, "lin_o(prod(lin_l(x_l), lin_r(x_r)))");
+    register_ops(m);                                   // the linears and the PaiNN layers (torch_ops.cpp)
     // codegen_tensops_cuda (codegen_tensops.cpp:2001-2010): the gradients arrive as positional arguments
     m.def("bee_fwd_cuda", &bee_fwd);
     m.def("bee_bwl_cuda", [](const at::Tensor& r_0, const at::Tensor& r_1, const at::Tensor& r_2, const py::args& dys) {

@@ -1,0 +1,626 @@
+// Host side of the linear maps and of the PaiNN layers in C++: what ops.py and painn.py call per forward pass.  A call
+// checks its operands, allocates outputs, looks packed weights up and enqueues kernels of libmanagan_hip.so on torch's
+// current stream: about 3 us per launch, where the same steps through ctypes took about 12, which is what a network of
+// node-sized launches was bound by.  No arithmetic happens here.
+#include "torch_common.hpp"
+
+#include <atomic>
+#include <map>
+#include <mutex>
+#include <tuple>
+
+using namespace mgt;
+
+namespace {
+
+enum { kActNone = 0, kActSilu = 1, kActLeaky = 2 };
+enum { kModeFp32 = 0, kModeBf16x3 = 1, kModeF16x2 = 2 };
+
+std::atomic<int64_t> g_epoch{0};        // of invalidate_weight_caches
+
+// ------------------------------------------------------------------ tensors derived from weights, kept per version
+// An entry belongs to a tensor OBJECT (a weak reference keeps the address from being reused) and its version counter;
+// a view (the transposed weight of an input-gradient product is a fresh view of the parameter) is kept under the tensor
+// it views.  Inference tensors have no version counter: nothing is kept for them.
+template <typename Value>
+class WeightCache {
+public:
+    using Key = std::tuple<const void*, int, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t>;
+    struct Slot {
+        c10::weak_intrusive_ptr<c10::TensorImpl> owner;
+        uint32_t version;
+        const void* data;
+        int64_t epoch;
+        Value value;
+    };
+
+    template <typename Make>
+    Value get(const at::Tensor& W, int kind, int64_t extra, Make&& make) {
+        const at::Tensor owner = W.is_view() ? at::Tensor(W._base()) : W;
+        if (owner.is_inference()) return make();
+        c10::TensorImpl* impl = owner.unsafeGetTensorImpl();
+        const Key key{impl, kind, extra, W.storage_offset(), W.size(0), W.size(-1), W.stride(0), W.stride(-1)};
+        const uint32_t version = impl->version_counter().current_version();
+        const void* data = owner.data_ptr();
+        const int64_t epoch = g_epoch.load();
+        {
+            std::lock_guard<std::mutex> lock(mutex_);
+            auto it = slots_.find(key);
+            if (it != slots_.end() && it->second.version == version && it->second.data == data && it->second.epoch == epoch)
+                return it->second.value;
+        }
+        Value v = make();
+        std::lock_guard<std::mutex> lock(mutex_);
+        if (++inserts_ % 64 == 0 || slots_.size() > 8192)          // drop what belonged to tensors that are gone
+            for (auto it = slots_.begin(); it != slots_.end();) it = it->second.owner.expired() ? slots_.erase(it) : std::next(it);
+        slots_.erase(key);
+        slots_.emplace(key, Slot{c10::weak_intrusive_ptr<c10::TensorImpl>(owner.getIntrusivePtr()), version, data, epoch, v});
+        return v;
+    }
+
+private:
+    std::mutex mutex_;
+    std::map<Key, Slot> slots_;
+    int64_t inserts_ = 0;
+};
+
+template <typename Value>
+WeightCache<Value>& cache() {
+    static WeightCache<Value>* c = new WeightCache<Value>;     // never destroyed: the allocator may be gone by then
+    return *c;
+}
+
+at::Tensor bytes_like(const at::Tensor& t, size_t n) {
+    return at::empty({(int64_t)n}, t.options().dtype(at::kByte).requires_grad(false));
+}
+at::Tensor floats(const at::Tensor& like, at::IntArrayRef shape) {
+    return at::empty(shape, like.options().requires_grad(false));
+}
+
+// fp16 hi / lo planes + inverse row scales of W, its reduction dimension zero-padded to k_pad
+at::Tensor packed_f16x2(const at::Tensor& W, int64_t k_pad) {
+    return cache<at::Tensor>().get(W, 2, k_pad, [&] {
+        size_t n = 0;
+        check(mg_linear_f16x2_packed_weight_bytes((int)k_pad, (int)W.size(0), &n));
+        at::Tensor p = bytes_like(W, n);
+        check(mg_linear_f16x2_pack_weight_padded(fp(W), W.stride(0), W.stride(1), (int)W.size(1), (int)W.size(0), (int)k_pad,
+                                                 p.data_ptr(), stream_of(W)));
+        return p;
+    });
+}
+at::Tensor packed_bf16x3(const at::Tensor& W) {
+    return cache<at::Tensor>().get(W, 1, 0, [&] {
+        size_t n = 0;
+        check(mg_linear_packed_weight_bytes((int)W.size(1), (int)W.size(0), &n));
+        at::Tensor p = bytes_like(W, n);
+        check(mg_linear_pack_weight(fp(W), W.stride(0), W.stride(1), (int)W.size(1), (int)W.size(0), p.data_ptr(), stream_of(W)));
+        return p;
+    });
+}
+at::Tensor packed_weight(const at::Tensor& W, bool f16) {
+    TORCH_CHECK(W.is_cuda() && W.scalar_type() == at::kFloat && W.dim() == 2, "W must be a float32 CUDA matrix");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(W.device());
+    return f16 ? packed_f16x2(W, W.size(1)) : packed_bf16x3(W);
+}
+
+// (max_o sum_i |W[o, i]|, max_o |bias[o]|): |act(x W^T + bias)| <= |x|max * first + second for |act(z)| <= |z|; read back
+// once per version of the parameters
+std::pair<float, float> norms_of(const at::Tensor& W, const OptTensor& bias) {
+    auto read = [](const at::Tensor& t) { return t.item<float>(); };
+    auto weight = cache<float>().get(W, 3, 0, [&] {
+        c10::InferenceMode off(false);
+        at::NoGradGuard no_grad;
+        return read(W.detach().abs().sum(1).amax()) * (1.0f + 1e-6f);
+    });
+    float b = 0.f;
+    if (bias.has_value())
+        b = cache<float>().get(*bias, 4, 0, [&] {
+            c10::InferenceMode off(false);
+            at::NoGradGuard no_grad;
+            return read(bias->detach().abs().amax()) * (1.0f + 1e-6f);
+        });
+    return {weight, b};
+}
+
+// ------------------------------------------------------------------ linear maps
+// upper bounds of the row maxima of |x|: mul * base + add, base (rows / rows_per, parts) or (1, parts)
+struct Bound {
+    OptTensor base;
+    float mul = 1.f, add = 0.f;
+    int64_t rows_per = 1;
+};
+
+bool f16x2_takes(int64_t rows, int64_t dim_in, int64_t dim_out, const at::Tensor& x) {
+    return dim_in % 32 == 0 && dim_in >= 64 && dim_out >= 8 && rows >= 1 && aligned16(x);
+}
+
+at::Tensor row_absmax(const at::Tensor& x) {
+    check_input(x, "x");
+    TORCH_CHECK(x.dim() == 2, "x must have two dims");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    at::Tensor out = floats(x, {x.size(0), 1});
+    check(mg_row_absmax(fp(x), x.size(0), (int)x.size(1), fp(out), stream_of(x)));
+    return out;
+}
+
+int64_t rowmax_parts(int64_t rows, int64_t dim_in, int64_t dim_out, bool sequential) {
+    return sequential ? mg_tensor_linear_f16x2_rowmax_parts_sequential(rows, (int)dim_in, (int)dim_out)
+                      : mg_tensor_linear_f16x2_rowmax_parts(rows, (int)dim_in, (int)dim_out);
+}
+
+// x (rows, k) plain rows; y preallocated
+void run_f16x2(const at::Tensor& W, int64_t k, const float* x, int64_t rows, const Bound& b, const OptTensor& bias, int act,
+               bool accumulate, int out_comps, at::Tensor& y, at::Tensor* ymax, bool sequential, int64_t bias_rows = -1) {
+    const at::Tensor planes = packed_f16x2(W, k);
+    const at::Tensor& base = *b.base;
+    mg_f16x2_linear a{};
+    a.packed_W = planes.data_ptr();
+    a.x = x;
+    a.x_rowmax = fp(base);
+    a.x_rowmax_parts = (int)base.size(1);
+    a.x_rowmax_stride = base.size(0) > 1 || rows == b.rows_per ? base.size(1) : 0;
+    a.x_rows_per_bound = b.rows_per;
+    a.bound_mul = b.mul;
+    a.bound_add = b.add;
+    a.rows = rows;
+    a.dim_in = (int)k;
+    a.dim_out = (int)W.size(0);
+    a.bias = fp(bias);
+    a.bias_rows = bias_rows < 0 ? rows : bias_rows;
+    a.act = act;
+    a.accumulate = accumulate;
+    a.out_comps = out_comps;
+    a.sequential = sequential;
+    a.y = fp(y);
+    a.y_rowmax = ymax ? fp(*ymax) : nullptr;
+    check(mg_tensor_linear_f16x2_run(&a, stream_of(y)));
+}
+
+void check_bound(const at::Tensor& b, int64_t rows, int64_t rows_per) {
+    check_input(b, "x_rowmax");
+    TORCH_CHECK(b.dim() == 2 && (b.size(0) == 1 || b.size(0) * rows_per == rows),
+                "x_rowmax must be (rows / rows_per_bound, parts) or (1, parts)");
+}
+
+// y = act(x W^T + bias) for plain rows through the two-piece fp16 split
+std::tuple<at::Tensor, OptTensor> linear_f16x2(const at::Tensor& W, const at::Tensor& x, const OptTensor& x_rowmax, double mul,
+                                               double add, const OptTensor& bias, int act, const OptTensor& out,
+                                               bool accumulate, int out_comps, bool want_rowmax, int64_t rows_per,
+                                               bool sequential) {
+    check_input(x, "x");
+    TORCH_CHECK(x.dim() == 2 && W.dim() == 2 && x.size(1) == W.size(1), "expected x (rows, dim_in) and W (dim_out, dim_in)");
+    const int64_t rows = x.size(0), dim_in = W.size(1), dim_out = W.size(0);
+    Bound b{x_rowmax.has_value() ? x_rowmax : OptTensor(row_absmax(x)), (float)mul, (float)add, rows_per};
+    check_bound(*b.base, rows, rows_per);
+    if (bias.has_value()) {
+        check_input(*bias, "bias");
+        TORCH_CHECK(bias->numel() == dim_out, "bias size mismatch");
+    }
+    TORCH_CHECK(rows % out_comps == 0, "rows must be a multiple of out_comps");
+    TORCH_CHECK(!want_rowmax || out_comps == 1, "row maxima are only produced for out_comps == 1");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    at::Tensor y;
+    if (out.has_value()) {
+        check_input(*out, "out");
+        TORCH_CHECK(out->numel() == rows * dim_out, "out has wrong size");
+        y = *out;
+    } else if (out_comps == 1) {
+        y = floats(x, {rows, dim_out});
+    } else {
+        y = floats(x, {rows / out_comps, dim_out, out_comps});
+    }
+    at::Tensor ymax;
+    if (want_rowmax) ymax = floats(x, {rows, rowmax_parts(rows, dim_in, dim_out, sequential)});
+    run_f16x2(W, dim_in, fp(x), rows, b, bias, act, accumulate, out_comps, y, want_rowmax ? &ymax : nullptr, sequential);
+    return {y, want_rowmax ? OptTensor(ymax) : OptTensor()};
+}
+
+// x (rows, dim, comps) -> one plain row per (row, comp), channels zero-padded to `pad`, and the row maxima
+std::pair<at::Tensor, at::Tensor> components_to_rows(const at::Tensor& x, int64_t rows, int64_t dim, int T, int64_t pad) {
+    at::Tensor x2 = floats(x, {rows * T, pad}), m = floats(x, {rows * T, 1});
+    check(mg_components_to_rows(fp(x), rows, (int)dim, T, (int)pad, fp(x2), fp(m), stream_of(x)));
+    return {x2, m};
+}
+
+bool power_of_two(int64_t v) { return v > 0 && (v & (v - 1)) == 0; }
+
+// rows x components from which a tensor linear goes through plain component rows and the split-fp16 kernels; in sequential
+// order the old crossover stays: an element's order of summation must not change with the number of rows in between
+constexpr int64_t kComponentRows = 960, kComponentRowsSequential = 32768;
+
+std::tuple<at::Tensor, OptTensor> linear_fwd(int64_t inds, const at::Tensor& W, const at::Tensor& x, const OptTensor& bias,
+                                             int act, const OptTensor& out, bool accumulate, int x_layout, int y_layout,
+                                             const OptTensor& row_bound, double mul, double add, int64_t rows_per,
+                                             bool want_rowmax, const OptTensor& x2_given, const OptTensor& x2max_given,
+                                             bool sequential) {
+    TORCH_CHECK(W.is_cuda(), "W must be a CUDA tensor");
+    check_input(x, "x");
+    TORCH_CHECK(W.scalar_type() == at::kFloat, "W must be float32");
+    TORCH_CHECK(W.dim() == 2, "expected W to be a matrix (2 dims)");
+    TORCH_CHECK(inds >= 0 && inds <= 2,
+                "tensor_linear currently only supports a number of indices up to 2. go edit the code to add more (easy with "
+                "copy/paste).");
+    const int64_t dim_out = W.size(0), dim_in = W.size(1);
+    const int T = inds == 0 ? 1 : inds == 1 ? 3 : 9;
+    int64_t batch_dims;
+    if (x_layout == 0) {
+        batch_dims = x.dim() - (1 + inds);
+        TORCH_CHECK(batch_dims >= 0, "x has too few dims");
+        TORCH_CHECK(x.size(batch_dims) == dim_in, "channel dim size mismatch for x");
+        for (int64_t i = batch_dims + 1; i <= batch_dims + inds; i++)
+            TORCH_CHECK(x.size(i) == 3, "expected tensor index dim to be 3d for input x");
+    } else {
+        batch_dims = x.dim() - 2;
+        TORCH_CHECK(batch_dims >= 0 && x.size(-1) == dim_in && x.size(-2) == T,
+                    "component-major x must have shape (..., 3^inds, dim_in)");
+    }
+    std::vector<int64_t> y_shape(x.sizes().begin(), x.sizes().begin() + batch_dims);
+    int64_t rows = 1;
+    for (int64_t d : y_shape) rows *= d;
+    if (y_layout == 0) {
+        y_shape.push_back(dim_out);
+        for (int64_t k = 0; k < inds; k++) y_shape.push_back(3);
+    } else {
+        y_shape.push_back(T);
+        y_shape.push_back(dim_out);
+    }
+    if (bias.has_value()) {
+        check_input(*bias, "bias");
+        TORCH_CHECK(bias->numel() == dim_out, "bias size mismatch");
+    }
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    at::Tensor y;
+    if (out.has_value()) {
+        check_input(*out, "out");
+        TORCH_CHECK(out->sizes() == at::IntArrayRef(y_shape), "out has wrong shape");
+        y = *out;
+    } else {
+        y = floats(x, y_shape);
+    }
+    const int mode = mg_get_linear_mode();
+    const bool plain_rows = inds == 0 || x_layout == 1;
+    const int64_t R = rows * T;
+    const int out_comps = inds == 0 || y_layout == 1 ? 1 : T;
+    at::Tensor ymax;
+    const bool emit = want_rowmax && out_comps == 1 && !accumulate;
+    auto rowmax_buffer = [&](int64_t k) {
+        if (emit) ymax = floats(x, {R, rowmax_parts(R, k, dim_out, sequential)});
+        return emit ? &ymax : nullptr;
+    };
+    const int64_t k_pad = (dim_in + 31) / 32 * 32;
+    if (mode == kModeF16x2 && inds > 0 && x_layout == 0 && R >= (sequential ? kComponentRowsSequential : kComponentRows) &&
+        (sequential || dim_in > 8) && dim_out >= 64 && !row_bound.has_value() &&
+        (y_layout == 1 || !(want_rowmax || accumulate || bias.has_value() || act != kActNone))) {
+        // (row, chan, comp) -> (row, comp, chan) rows, then the plain-row matrix path: its component-major output is
+        // written at the full store rate, and with the reference's output layout its component epilogue still beats the
+        // generic kernel (61 against 104 us for 16384 x 128 x 3 -> 384, 9 against 22 us for 337 x 128 x 3 -> 384)
+        at::Tensor x2, x2max;
+        if (x2_given.has_value() && x2_given->dim() == 2 && x2_given->size(0) == R && x2_given->size(1) == k_pad) {
+            x2 = *x2_given;
+            x2max = *x2max_given;
+        } else if (k_pad <= 256 && power_of_two(k_pad)) {
+            std::tie(x2, x2max) = components_to_rows(x, rows, dim_in, T, k_pad);
+        } else {
+            at::Tensor xt = x.reshape({rows, dim_in, T}).transpose(1, 2);
+            xt = k_pad != dim_in ? at::constant_pad_nd(xt, {0, k_pad - dim_in}) : xt.contiguous();
+            x2 = xt.reshape({R, k_pad});
+            x2max = row_absmax(x2);
+        }
+        run_f16x2(W, k_pad, fp(x2), R, Bound{x2max}, bias, act, accumulate, out_comps, y, rowmax_buffer(k_pad), sequential);
+    } else if (plain_rows && mode == kModeF16x2 && f16x2_takes(R, dim_in, dim_out, x) && (!sequential || R >= 256)) {
+        Bound b{row_bound, (float)mul, (float)add, rows_per};
+        if (row_bound.has_value()) {
+            TORCH_CHECK(row_bound->dim() == 2 && (row_bound->size(0) * rows_per == R || row_bound->size(0) == 1),
+                        "row_bound must be (rows / rows_per_bound, parts)");
+        } else {
+            b = Bound{row_absmax(x.reshape({R, dim_in}))};
+        }
+        run_f16x2(W, dim_in, fp(x), R, b, bias, act, accumulate, out_comps, y, rowmax_buffer(dim_in), sequential);
+    } else if (mode == kModeBf16x3 && plain_rows && dim_in % 32 == 0 && dim_in >= 64 && dim_out >= 64 && R >= 1024 &&
+               aligned16(x)) {
+        check(mg_tensor_linear_packed(packed_bf16x3(W).data_ptr(), fp(x), R, (int)dim_in, (int)dim_out, fp(bias), act,
+                                      accumulate, out_comps, fp(y), stream_of(x)));
+    } else {
+        check(mg_tensor_linear_layout((int)inds, fp(W), W.stride(0), W.stride(1), fp(x), rows, (int)dim_in, (int)dim_out,
+                                      fp(bias), act, accumulate, x_layout, y_layout, fp(y), stream_of(x)));
+    }
+    return {y, ymax.defined() ? OptTensor(ymax) : OptTensor()};
+}
+
+// dW (and with want_bias db): see ops.tensor_linear_wgrad
+std::tuple<at::Tensor, OptTensor> linear_wgrad(int64_t inds, const at::Tensor& dy, const at::Tensor& x,
+                                               const OptTensor& dy_bound, const OptTensor& x_bound, bool want_bias) {
+    check_input(dy, "dy");
+    check_input(x, "x");
+    TORCH_CHECK(!want_bias || inds == 0, "the bias gradient is defined for plain rows only");
+    const int64_t batch_dims = x.dim() - (1 + inds);
+    const int64_t dim_in = x.size(batch_dims), dim_out = dy.size(batch_dims);
+    int64_t rows = 1;
+    for (int64_t i = 0; i < batch_dims; i++) rows *= x.size(i);
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    const int T = inds == 0 ? 1 : inds == 1 ? 3 : 9;
+    const int mode = mg_get_linear_mode();
+    at::Tensor dW = floats(x, {dim_out, dim_in});
+    auto workspace = [&](int64_t n_rows, int64_t n_in, int64_t n_out) {
+        size_t n = 0;
+        check(mg_tensor_linear_wgrad_workspace_bytes(n_rows, (int)n_in, (int)n_out, &n));
+        return bytes_like(x, n);
+    };
+    OptTensor db;
+    if (inds == 0 && mode == kModeF16x2 && aligned16(x) && aligned16(dy) &&
+        mg_tensor_linear_wgrad_f16x2_supported(rows, (int)dim_in, (int)dim_out)) {
+        if (dy_bound.has_value()) check_input(*dy_bound, "dy_bound");
+        if (x_bound.has_value()) check_input(*x_bound, "x_bound");
+        at::Tensor bias_grad;
+        if (want_bias) bias_grad = floats(x, {dim_out});
+        at::Tensor ws = workspace(rows, dim_in, dim_out);
+        check(mg_tensor_linear_wgrad_f16x2(fp(dy), fp(x), fp(dy_bound), dy_bound.has_value() ? dy_bound->numel() : 0, fp(x_bound),
+                                           x_bound.has_value() ? x_bound->numel() : 0, rows, (int)dim_in, (int)dim_out,
+                                           ws.data_ptr(), fp(dW), want_bias ? fp(bias_grad) : nullptr, stream_of(x)));
+        if (want_bias) db = bias_grad;
+    } else if (inds > 0 && mode == kModeF16x2 && rows * T >= 4096 && std::max(dim_in, dim_out) <= 256) {
+        // (row, chan, comp) -> one plain row per (row, comp), channels zero-padded to a power of two: the sum over rows
+        // and components is then the plain-row weight gradient, on the matrix cores; the transposition also yields the
+        // row maxima the kernel scales by
+        auto pad_of = [](int64_t d) {
+            int64_t p = 32;
+            while (p < d) p *= 2;
+            return p;
+        };
+        const int64_t o_pad = pad_of(dim_out), i_pad = pad_of(dim_in);
+        auto [dy2, dy2max] = components_to_rows(dy, rows, dim_out, T, o_pad);
+        auto [x2, x2max] = components_to_rows(x, rows, dim_in, T, i_pad);
+        at::Tensor ws = workspace(rows * T, i_pad, o_pad);
+        at::Tensor padded = o_pad == dim_out && i_pad == dim_in ? dW : floats(x, {o_pad, i_pad});
+        check(mg_tensor_linear_wgrad_f16x2(fp(dy2), fp(x2), fp(dy2max), rows * T, fp(x2max), rows * T, rows * T, (int)i_pad,
+                                           (int)o_pad, ws.data_ptr(), fp(padded), nullptr, stream_of(x)));
+        if (o_pad != dim_out || i_pad != dim_in) dW = padded.slice(0, 0, dim_out).slice(1, 0, dim_in).contiguous();
+    } else {
+        at::Tensor ws = workspace(rows, dim_in, dim_out);
+        check(mg_tensor_linear_wgrad((int)inds, fp(dy), fp(x), rows, (int)dim_in, (int)dim_out, ws.data_ptr(), fp(dW),
+                                     stream_of(x)));
+        if (want_bias) db = dy.reshape({-1, dim_out}).sum(0);
+    }
+    return {dW, db};
+}
+
+at::Tensor silu_order(const at::Tensor& z, int order, const OptTensor& mul) {
+    check_input(z, "z");
+    if (mul.has_value()) {
+        check_input(*mul, "mul");
+        TORCH_CHECK(mul->sizes() == z.sizes(), "mul must have the shape of z");
+    }
+    TORCH_CHECK(order >= 0 && order <= 4, "silu_order: order must be in 0..4");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(z.device());
+    at::Tensor out = floats(z, z.sizes());
+    check(mg_silu_order(fp(z), fp(mul), z.numel(), order, fp(out), stream_of(z)));
+    return out;
+}
+
+// ------------------------------------------------------------------ MLPs (inference)
+using Tensors = std::vector<at::Tensor>;
+
+// a chain of linears with fused bias and activation; the row bounds the split-fp16 layers scale by travel as
+// mul * base + add through the layers' norms, so that only the first layer ever looks at the data for them
+at::Tensor chain(at::Tensor h, const Tensors& W, const Tensors& b, const std::vector<int>& act, Bound bound) {
+    for (size_t k = 0; k < W.size(); k++) {
+        const int64_t rows = h.size(0), dim_in = W[k].size(1), dim_out = W[k].size(0);
+        at::Tensor y = floats(h, {rows, dim_out});
+        const OptTensor bias(b[k]);
+        if (rows == 0) {
+            h = y;
+            continue;
+        }
+        if (mg_get_linear_mode() == kModeF16x2 && f16x2_takes(rows, dim_in, dim_out, h)) {
+            if (!bound.base.has_value()) bound = Bound{row_absmax(h)};
+            run_f16x2(W[k], dim_in, fp(h), rows, bound, bias, act[k], false, 1, y, nullptr, false);
+        } else {
+            y = std::get<0>(linear_fwd(0, W[k], h, bias, act[k], OptTensor(y), false, 0, 0, OptTensor(), 1, 0, 1, false,
+                                       OptTensor(), OptTensor(), false));
+        }
+        if (bound.base.has_value() && k + 1 < W.size()) {
+            const auto [l1, bmax] = norms_of(W[k], bias);
+            bound.mul *= l1;
+            bound.add = bound.add * l1 + bmax;
+        }
+        h = y;
+    }
+    return h;
+}
+
+void check_chain(const at::Tensor& x, const Tensors& W, const Tensors& b, const std::vector<int>& act) {
+    check_input(x, "x");
+    TORCH_CHECK(x.dim() == 2 && W.size() == b.size() && W.size() == act.size() && !W.empty(), "linear_chain: bad arguments");
+    int64_t dim = x.size(1);
+    for (size_t k = 0; k < W.size(); k++) {
+        TORCH_CHECK(W[k].is_cuda() && W[k].scalar_type() == at::kFloat && W[k].dim() == 2 && W[k].size(1) == dim,
+                    "linear_chain: weights must be float32 CUDA matrices that follow each other");
+        check_input(b[k], "bias");
+        TORCH_CHECK(b[k].numel() == W[k].size(0), "bias size mismatch");
+        dim = W[k].size(0);
+    }
+}
+
+at::Tensor linear_chain(const at::Tensor& x, const Tensors& W, const Tensors& b, const std::vector<int>& act,
+                        const OptTensor& bound, double mul, double add) {
+    check_chain(x, W, b, act);
+    if (bound.has_value()) check_bound(*bound, x.size(0), 1);
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    return chain(x, W, b, act, Bound{bound, (float)mul, (float)add});
+}
+
+const std::vector<int> kSiluMlp{kActSilu, kActSilu, kActNone};
+
+// ------------------------------------------------------------------ PaiNN layers (inference)
+// Update.forward: x_a (batch, nodes, n), x_v (batch, nodes, n, 3); W_lrv (3n, n) the stacked l, r, v maps
+std::tuple<at::Tensor, at::Tensor> painn_update(const at::Tensor& x_a, const at::Tensor& x_v, const at::Tensor& W_lrv,
+                                                const Tensors& W, const Tensors& b, int groups, const at::Tensor& gamma,
+                                                const at::Tensor& beta, double eps, bool residual) {
+    check_input(x_a, "x_a");
+    check_input(x_v, "x_v");
+    TORCH_CHECK(x_a.dim() == 3 && x_v.dim() == 4 && x_v.size(3) == 3 && x_v.size(2) == x_a.size(2) &&
+                    x_v.size(0) == x_a.size(0) && x_v.size(1) == x_a.size(1),
+                "x_a must have shape (batch, nodes, n) and x_v (batch, nodes, n, 3)");
+    const int64_t B = x_a.size(0), N = x_a.size(1), n = x_a.size(2), rows = B * N;
+    TORCH_CHECK(W_lrv.size(0) == 3 * n && W_lrv.size(1) == n, "W_lrv must have shape (3n, n)");
+    check_input(gamma, "gamma");
+    check_input(beta, "beta");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x_a.device());
+    const at::Tensor flat_v = x_v.reshape({rows, n, 3});
+    // component-major (rows, 3, 3n): the GEMM stores whole rows, the two kernels below read with unit stride
+    const at::Tensor lrv = std::get<0>(linear_fwd(1, W_lrv, flat_v, OptTensor(), kActNone, OptTensor(), false, 0, 1, OptTensor(),
+                                                  1, 0, 1, false, OptTensor(), OptTensor(), false));
+    at::Tensor ip = floats(x_a, {rows, n}), cat = floats(x_a, {rows, 2 * n}), cat_max;
+    if (n <= 256) cat_max = floats(x_a, {rows, 1});
+    const mg_stream_t st = stream_of(x_a);
+    check(mg_painn_update_pre(fp(lrv), 1, fp(x_a), rows, (int)n, fp(ip), fp(cat), n <= 256 ? fp(cat_max) : nullptr, st));
+    check_chain(cat, W, b, kSiluMlp);
+    at::Tensor y = chain(cat, W, b, kSiluMlp, Bound{n <= 256 ? OptTensor(cat_max) : OptTensor()});          // (rows, 3n)
+    at::Tensor out_a = floats(x_a, x_a.sizes()), out_v = floats(x_v, x_v.sizes());
+    size_t scratch_bytes = 0;
+    check(mg_group_norm_scratch_bytes((int)B, groups, &scratch_bytes));
+    at::Tensor scratch = bytes_like(x_a, std::max<size_t>(scratch_bytes, 8));
+    check(mg_group_norm(1, fp(ip), n, fp(y) + n, 3 * n, (int)B, (int)N, (int)n, groups, 1, (float)eps, fp(gamma), fp(beta),
+                        fp(y) + 2 * n, 3 * n, residual ? fp(x_a) : nullptr, scratch.data_ptr(), fp(out_a), st));
+    check(mg_painn_update_vec(fp(lrv), 1, fp(y), residual ? fp(x_v) : nullptr, rows, (int)n, fp(out_v), st));
+    return {out_a, out_v};
+}
+
+struct MessageArgs {
+    const at::Tensor &row_ptr, &dst, &r_ij, &x_a, &x_v;
+    int64_t B, N, n, rows, E;
+};
+MessageArgs message_args(const at::Tensor& row_ptr, const at::Tensor& dst, const at::Tensor& r_ij, const at::Tensor& x_a,
+                         const at::Tensor& x_v) {
+    check_input(row_ptr, "row_ptr", at::kInt);
+    check_input(dst, "dst", at::kInt);
+    check_input(r_ij, "r_ij");
+    check_input(x_a, "x_a");
+    check_input(x_v, "x_v");
+    TORCH_CHECK(x_a.dim() == 3 && x_v.dim() == 4 && x_v.size(3) == 3 && x_v.size(2) == x_a.size(2) &&
+                    x_v.size(0) == x_a.size(0) && x_v.size(1) == x_a.size(1),
+                "x_a must have shape (batch, nodes, n) and x_v (batch, nodes, n, 3)");
+    MessageArgs m{row_ptr, dst, r_ij, x_a, x_v, x_a.size(0), x_a.size(1), x_a.size(2), x_a.size(0) * x_a.size(1), dst.numel()};
+    TORCH_CHECK(row_ptr.numel() == m.rows + 1, "row_ptr must have nodes+1 entries");
+    TORCH_CHECK(r_ij.dim() == 2 && r_ij.size(0) == m.E && r_ij.size(1) == 3, "r_ij must have shape (edges, 3)");
+    return m;
+}
+
+// The filter MLP on the encodings enc (rows, k) of a grid, all at most 1 in magnitude; where k exceeds the first layer's
+// input the encodings end in zero columns and the weight is padded likewise (a reduction the matrix path takes).
+at::Tensor filter_grid(const at::Tensor& enc, const at::Tensor& unit, const Tensors& W, const Tensors& b) {
+    check_input(enc, "enc");
+    check_input(unit, "unit");
+    const int64_t k = enc.size(1), rows = enc.size(0);
+    if (k == W[0].size(1)) {
+        check_chain(enc, W, b, kSiluMlp);
+        return chain(enc, W, b, kSiluMlp, Bound{OptTensor(unit)});
+    }
+    TORCH_CHECK(k > W[0].size(1) && k % 32 == 0 && mg_get_linear_mode() == kModeF16x2 && aligned16(enc),
+                "filter_grid: encodings of a wrong width");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(enc.device());
+    at::Tensor h = floats(enc, {rows, W[0].size(0)});
+    const OptTensor b0(b[0]);
+    run_f16x2(W[0], k, fp(enc), rows, Bound{OptTensor(unit)}, b0, kActSilu, false, 1, h, nullptr, false);
+    const auto [l1, bmax] = norms_of(W[0], b0);
+    check_chain(h, {W[1], W[2]}, {b[1], b[2]}, {kActSilu, kActNone});
+    return chain(h, {W[1], W[2]}, {b[1], b[2]}, {kActSilu, kActNone}, Bound{OptTensor(unit), l1, bmax});
+}
+
+// Message.forward with the filter interpolated from its grid, which is evaluated here: enc (rows, k) the grid's
+// encodings, k the first layer's reduction dimension after zero padding.  sliced: the grid in LDS, the last layer of
+// mlp_actv given with its rows slice by slice.
+std::tuple<at::Tensor, at::Tensor> painn_message_grid(const at::Tensor& row_ptr, const at::Tensor& dst, const at::Tensor& r_ij,
+                                                      const OptTensor& order, const at::Tensor& x_a, const at::Tensor& x_v,
+                                                      const Tensors& W_actv, const Tensors& b_actv, const OptTensor& enc,
+                                                      const OptTensor& unit, const Tensors& W_dist, const Tensors& b_dist,
+                                                      const OptTensor& table_given, double period, double epsilon, bool sliced,
+                                                      bool residual) {
+    const MessageArgs m = message_args(row_ptr, dst, r_ij, x_a, x_v);
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x_a.device());
+    const at::Tensor flat_a = x_a.reshape({m.rows, m.n});
+    check_chain(flat_a, W_actv, b_actv, kSiluMlp);
+    const at::Tensor actv = chain(flat_a, W_actv, b_actv, kSiluMlp, Bound{});
+    TORCH_CHECK(actv.size(1) == 4 * m.n, "actv must have shape (nodes, 4n)");
+    at::Tensor table;
+    if (table_given.has_value()) {
+        check_input(*table_given, "table");
+        table = *table_given;
+    } else {
+        table = filter_grid(*enc, *unit, W_dist, b_dist);
+    }
+    TORCH_CHECK(table.dim() == 2 && table.size(1) == 4 * m.n, "table must have shape (rows, 4n)");
+    if (order.has_value()) {
+        check_input(*order, "node_order", at::kInt);
+        TORCH_CHECK(order->numel() == m.rows, "node_order must have one entry per node");
+    }
+    const int* ord = order.has_value() ? order->data_ptr<int>() : nullptr;
+    at::Tensor out_a = floats(x_a, x_a.sizes()), out_v = floats(x_v, x_v.sizes());
+    const mg_stream_t st = stream_of(x_a);
+    const float *res_a = residual ? fp(x_a) : nullptr, *res_v = residual ? fp(x_v) : nullptr;
+    if (sliced) {
+        at::Tensor rec = floats(x_a, {m.E, 8});
+        check(mg_painn_edge_records(fp(r_ij), m.E, (int)table.size(0), (float)period, (float)epsilon, fp(rec), st));
+        check(mg_painn_table_message_sliced(row_ptr.data_ptr<int>(), dst.data_ptr<int>(), ord, m.rows, m.E, fp(rec), fp(table),
+                                            (int)table.size(0), fp(actv), fp(x_v), (int)m.n, res_a, res_v, fp(out_a), fp(out_v),
+                                            st));
+    } else {
+        check(mg_painn_table_message(row_ptr.data_ptr<int>(), dst.data_ptr<int>(), ord, m.rows, m.E, fp(r_ij), fp(table),
+                                     (int)table.size(0), (float)period, fp(actv), fp(x_v), (int)m.n, (float)epsilon, res_a,
+                                     res_v, fp(out_a), fp(out_v), st));
+    }
+    return {out_a, out_v};
+}
+
+// Message.forward with the filter MLP on every edge and the filter stored (few edges: the kernels that fold its layers into
+// the edge kernel are made for tiles of 256 edges)
+std::tuple<at::Tensor, at::Tensor> painn_message_edges(const at::Tensor& row_ptr, const at::Tensor& dst, const at::Tensor& r_ij,
+                                                       const at::Tensor& x_a, const at::Tensor& x_v, const Tensors& W_actv,
+                                                       const Tensors& b_actv, const at::Tensor& unit, const Tensors& W_dist,
+                                                       const Tensors& b_dist, double rmax, double epsilon, bool residual) {
+    const MessageArgs m = message_args(row_ptr, dst, r_ij, x_a, x_v);
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x_a.device());
+    const at::Tensor flat_a = x_a.reshape({m.rows, m.n});
+    check_chain(flat_a, W_actv, b_actv, kSiluMlp);
+    const at::Tensor actv = chain(flat_a, W_actv, b_actv, kSiluMlp, Bound{});
+    TORCH_CHECK(actv.size(1) == 4 * m.n && W_dist.size() == 3 && W_dist[2].size(0) == 4 * m.n, "weights must end in 4n rows");
+    const mg_stream_t st = stream_of(x_a);
+    const int64_t n_rbf = W_dist[0].size(1), hidden = W_dist[0].size(0);
+    at::Tensor filt;
+    const int64_t g = hidden / 4;
+    if (n_rbf <= 32 && hidden % 4 == 0 && g >= 1 && g <= 256 && 256 % g == 0) {
+        at::Tensor h = floats(x_a, {m.E, hidden});
+        check(mg_painn_radial_linear(fp(r_ij), m.E, (int)n_rbf, (float)rmax, fp(W_dist[0]), W_dist[0].stride(0),
+                                     W_dist[0].stride(1), fp(b_dist[0]), (int)hidden, kActSilu, fp(h), st));
+        const auto [l1, bmax] = norms_of(W_dist[0], OptTensor(b_dist[0]));
+        filt = chain(h, {W_dist[1], W_dist[2]}, {b_dist[1], b_dist[2]}, {kActSilu, kActNone}, Bound{OptTensor(unit), l1, bmax});
+    } else {
+        at::Tensor enc = floats(x_a, {m.E, n_rbf});
+        check(mg_painn_radial_encode(fp(r_ij), m.E, (int)n_rbf, (float)rmax, fp(enc), st));
+        check_chain(enc, W_dist, b_dist, kSiluMlp);
+        filt = chain(enc, W_dist, b_dist, kSiluMlp, Bound{OptTensor(unit)});
+    }
+    at::Tensor out_a = floats(x_a, x_a.sizes()), out_v = floats(x_v, x_v.sizes());
+    check(mg_painn_message(row_ptr.data_ptr<int>(), dst.data_ptr<int>(), nullptr, m.rows, m.E, fp(r_ij), fp(filt), fp(actv),
+                           fp(x_v), (int)m.n, (float)epsilon, residual ? fp(x_a) : nullptr, residual ? fp(x_v) : nullptr,
+                           fp(out_a), fp(out_v), st));
+    return {out_a, out_v};
+}
+
+}  // namespace
+
+void register_ops(pybind11::module_& m) {
+    namespace py = pybind11;
+    m.def("invalidate_weight_caches", [] { g_epoch.fetch_add(1); });
+    m.def("packed_weight", &packed_weight);
+    m.def("row_absmax", &row_absmax);
+    m.def("linear_f16x2", &linear_f16x2);
+    m.def("linear_fwd", &linear_fwd);
+    m.def("linear_wgrad", &linear_wgrad);
+    m.def("silu_order", &silu_order);
+    m.def("linear_chain", &linear_chain);
+    m.def("filter_grid", &filter_grid);
+    m.def("painn_update", &painn_update);
+    m.def("painn_message_grid", &painn_message_grid);
+    m.def("painn_message_edges", &painn_message_edges);
+}

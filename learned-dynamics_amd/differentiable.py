@@ -121,12 +121,12 @@ def jvp(f, primals, tangents, create_graph=True, strict=False):
         return unpack(out)
 
 
-def linear(lin, x, x_bound=None, want_bound=False):
+def linear(lin, x, x_bound=None, want_bound=False, sequential=True):
     """nn.Linear through the tensor_linear kernels (weight and input gradients are kernels too).  x_bound / want_bound:
-    row maxima handed from one layer to the next (tensor_products.tensor_linear)."""
+    row maxima handed from one layer to the next (tensor_products.tensor_linear).  sequential: see _TensorLinearFn."""
     lead = x.shape[:-1]
     out = tensor_linear(0, lin.weight, x.reshape(-1, x.shape[-1]).contiguous(), bias=lin.bias, x_bound=x_bound,
-                        want_bound=want_bound)
+                        want_bound=want_bound, sequential=sequential)
     if want_bound:
         return out[0].reshape(*lead, -1), out[1]
     return out.reshape(*lead, -1)
@@ -175,9 +175,9 @@ def mlp_silu(mlp, x):
     """painn.MLP: Linear, SiLU, Linear, SiLU, Linear (archs/meanflow_painn8.py:38-51).  |SiLU(z)| <= |z|: the row
     maxima that a layer's kernel emits for z bound the next layer's input."""
     L = mlp.layers
-    z, b = linear(L[0], x, want_bound=True)
-    z, b = linear(L[2], silu(z), x_bound=b, want_bound=True)
-    return linear(L[4], silu(z), x_bound=b)
+    z, b = linear(L[0], x, want_bound=True, sequential=False)
+    z, b = linear(L[2], silu(z), x_bound=b, want_bound=True, sequential=False)
+    return linear(L[4], silu(z), x_bound=b, sequential=False)
 
 
 def mlp_leaky(mlp, x):

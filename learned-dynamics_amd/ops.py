@@ -15,6 +15,7 @@ import torch
 from . import _lib as L
 
 _lib = L.load()
+_ext = L.load_torch_ext()       # the C++ host side of the hot calls (csrc/torch_ops.cpp)
 
 BEE_ORDER = ("000", "110", "220", "011", "101", "121", "211", "022", "202", "112", "222", "111", "212")
 
@@ -512,17 +513,7 @@ SILU_MAX_ORDER = 4
 
 def silu_order(z, order, mul=None):
     """SiLU^(order)(z), elementwise, times mul if given (same shape); order 0 .. SILU_MAX_ORDER."""
-    _check_input(z, "z")
-    if mul is not None:
-        _check_input(mul, "mul")
-        if mul.shape != z.shape:
-            raise RuntimeError("mul must have the shape of z")
-    if not 0 <= int(order) <= SILU_MAX_ORDER:
-        raise RuntimeError(f"silu_order: order must be in 0..{SILU_MAX_ORDER}")
-    with _on(z.device):
-        out = torch.empty_like(z)
-        L.check(_lib.mg_silu_order(_p(z), _p(mul) if mul is not None else None, z.numel(), int(order), _p(out), _stream()))
-    return out
+    return _ext.silu_order(z, int(order), mul)
 
 
 def bee_indexed_supported(chan):
@@ -916,7 +907,7 @@ def set_linear_mode(mode):
 
 
 def get_linear_mode():
-    return int(_lib.mg_get_linear_mode())
+    return _lib.mg_get_linear_mode()
 
 
 _cache_epoch = 0
@@ -928,6 +919,7 @@ def invalidate_weight_caches():
     version counter); a write that bypasses the counter (`param.data.mul_(...)`, a raw pointer) needs this call."""
     global _cache_epoch
     _cache_epoch += 1
+    _ext.invalidate_weight_caches()
 
 
 def tensor_version(t):
@@ -955,75 +947,53 @@ def derived_tensors():
         yield
 
 
-_packed_cache = {}
-
-
-def _packed(W, kind):
-    """Pre-split planes of W for the packed GEMM entry points.  Cached per tensor OBJECT (weak
-    reference) and version counter, so parameters are packed once and re-packed after an in-place
-    update; a new tensor that happens to reuse a freed address never hits a stale entry.  A view
-    (the transposed weight of every input-gradient GEMM is a fresh view object of the parameter) is
-    cached under the tensor it is a view of, with its offset, shape and strides."""
-    owner = W._base if W._base is not None else W
-    key = (id(owner), kind, int(W.storage_offset()), tuple(W.shape), tuple(W.stride()))
-    hit = _packed_cache.get(key)
-    version = tensor_version(owner)
-    if hit is not None and version >= 0 and hit[0]() is owner and hit[1] == version and hit[2] == owner.data_ptr():
-        return hit[3]
-    dim_out, dim_in = int(W.size(0)), int(W.size(1))
-    nbytes = ctypes.c_size_t(0)
-    size_fn, pack_fn = ((_lib.mg_linear_packed_weight_bytes, _lib.mg_linear_pack_weight) if kind == "bf16x3" else
-                        (_lib.mg_linear_f16x2_packed_weight_bytes, _lib.mg_linear_f16x2_pack_weight))
-    L.check(size_fn(dim_in, dim_out, ctypes.byref(nbytes)))
-    with _on(W.device):
-        packed = torch.empty(nbytes.value, dtype=torch.uint8, device=W.device)
-        L.check(pack_fn(_p(W), int(W.stride(0)), int(W.stride(1)), dim_in, dim_out, _p(packed), _stream()))
-    if len(_packed_cache) > 4096:
-        _packed_cache.clear()
-    # the entry (and the device memory of its planes) goes when the tensor it was packed from does
-    _packed_cache[key] = (weakref.ref(owner, lambda _, key=key: _packed_cache.pop(key, None)),
-                          version, owner.data_ptr(), packed)
-    return packed
-
-
-_padded_cache = {}
-
-
-def zero_padded_columns(W, k_pad):
-    """W (dim_out, dim_in) with zero columns appended up to k_pad; cached per parameter object and version."""
-    if int(W.size(1)) == k_pad:
-        return W
-    key = (id(W), k_pad)
-    hit = _padded_cache.get(key)
-    if hit is not None and hit[0]() is W and hit[1] == tensor_version(W) >= 0 and hit[2] == W.data_ptr():
-        return hit[3]
-    with derived_tensors():
-        Wp = torch.nn.functional.pad(W.detach(), (0, k_pad - int(W.size(1)))).contiguous()
-    if len(_padded_cache) > 256:
-        _padded_cache.clear()
-    _padded_cache[key] = (weakref.ref(W), tensor_version(W), W.data_ptr(), Wp)
-    return Wp
-
-
 def packed_weight(W):
-    """bf16x3 planes of W for mg_tensor_linear_packed."""
-    return _packed(W, "bf16x3")
+    """bf16x3 planes of W for mg_tensor_linear_packed, kept per tensor object and version (a view, such as the transposed
+    weight of an input-gradient GEMM, under the tensor it is a view of)."""
+    return _ext.packed_weight(W, False)
 
 
 def packed_weight_f16x2(W):
-    """fp16 hi/lo planes + per-row inverse scales of W for mg_tensor_linear_f16x2."""
-    return _packed(W, "f16x2")
+    """fp16 hi/lo planes + per-row inverse scales of W for mg_tensor_linear_f16x2, kept likewise."""
+    return _ext.packed_weight(W, True)
 
 
 def row_absmax(x):
     """(rows, dim) -> (rows, 1): max_i |x[r, i]|, the row bounds mg_tensor_linear_f16x2 scales by."""
-    _check_input(x, "x")
-    if x.dim() != 2:
-        raise RuntimeError("x must have two dims")
-    with _on(x.device):
-        out = torch.empty(x.size(0), 1, dtype=torch.float32, device=x.device)
-        L.check(_lib.mg_row_absmax(_p(x), int(x.size(0)), int(x.size(1)), _p(out), _stream()))
-    return out
+    return _ext.row_absmax(x)
+
+
+def linear_chain(x, weights, biases, acts, bound=None):
+    """act_k(.. act_1(x W_1^T + b_1) .. W_k^T + b_k), x (rows, dim) -> (rows, dim_out): an MLP's forward pass in one host
+    call.  bound: upper bounds of the row maxima of |x| ((rows, parts), (1, parts) or a ScaledBound) if the caller has
+    them; behind the first layer they follow from the layers' norms."""
+    return _ext.linear_chain(x, weights, biases, acts, *_bound_parts(bound))
+
+
+def filter_grid(enc, unit, weights, biases):
+    """The filter MLP (three linears with SiLU between) on encodings whose entries are at most 1 (unit: (1, 1) ones), whose
+    width may exceed the first layer's input by zero columns: (rows, dim) -> (rows, dim_out)."""
+    return _ext.filter_grid(enc, unit, weights, biases)
+
+
+def painn_update(x_a, x_v, W_lrv, weights, biases, gn, residual):
+    """Update.forward (archs/meanflow_painn8.py:63-75) in one host call: the stacked l, r, v maps, the MLP, the norm gn and
+    the gated vectors.  (out_a, out_v), with residual on top of x_a and x_v."""
+    return _ext.painn_update(x_a, x_v, W_lrv, weights, biases, gn.groups, gn.gamma, gn.beta, gn.epsilon, residual)
+
+
+def painn_message_grid(row_ptr, dst, r_ij, node_order, x_a, x_v, W_actv, b_actv, enc, unit, W_dist, b_dist, table, period,
+                       epsilon, sliced, residual):
+    """Message.forward (archs/meanflow_painn8.py:85-100) with the filter from its grid (evaluated here unless `table` holds
+    it) in one host call; sliced: painn_table_message_sliced with W_actv's last rows in the slices' order."""
+    return _ext.painn_message_grid(row_ptr, dst, r_ij, node_order, x_a, x_v, W_actv, b_actv, enc, unit, W_dist, b_dist, table,
+                                   period, epsilon, bool(sliced), residual)
+
+
+def painn_message_edges(row_ptr, dst, r_ij, x_a, x_v, W_actv, b_actv, W_dist, b_dist, rmax, epsilon, residual):
+    """Message.forward with the filter MLP on every edge and the filter stored, in one host call."""
+    return _ext.painn_message_edges(row_ptr, dst, r_ij, x_a, x_v, W_actv, b_actv, linear_in_unit_bound(x_a.device), W_dist,
+                                    b_dist, rmax, epsilon, residual)
 
 
 def linear_f64(W, bias, x, act=ACT_NONE):
@@ -1117,7 +1087,7 @@ def linear_out_bound_factors(W, bias):
 
 
 def f16x2_supported(rows, dim_in, dim_out, x):
-    return dim_in % 32 == 0 and dim_in >= 64 and dim_out >= 8 and rows >= 256 and x.data_ptr() % 16 == 0
+    return dim_in % 32 == 0 and dim_in >= 64 and dim_out >= 8 and rows >= 1 and x.data_ptr() % 16 == 0
 
 
 class ScaledBound:
@@ -1138,54 +1108,26 @@ class ScaledBound:
         return b * self.mul + self.add
 
 
+def _bound_parts(bound):
+    """(base, factor, offset) of row bounds given as a tensor, a ScaledBound or None."""
+    return (bound.base, bound.mul, bound.add) if isinstance(bound, ScaledBound) else (bound, 1.0, 0.0)
+
+
 def tensor_linear_f16x2(W, x, x_rowmax=None, bias=None, act=ACT_NONE, out=None, accumulate=False, out_comps=1,
                         want_rowmax=False, rows_per_bound=1):
     """y = act(x W^T + bias) for plain rows x (rows, dim_in) through the two-piece fp16 split.
     x_rowmax (rows, parts), or (1, parts) for one bound shared by all rows: upper bounds of the
     row maxima of |x| (None: computed here), or a ScaledBound of such an array.
     Returns y, or (y, y_rowmax) with want_rowmax=True."""
-    bound_mul, bound_add = 1.0, 0.0
-    if isinstance(x_rowmax, ScaledBound):
-        x_rowmax, bound_mul, bound_add = x_rowmax.base, x_rowmax.mul, x_rowmax.add
-    _check_input(x, "x")
-    if x.dim() != 2 or W.dim() != 2 or x.size(1) != W.size(1):
-        raise RuntimeError("expected x (rows, dim_in) and W (dim_out, dim_in)")
-    rows, dim_in, dim_out = int(x.size(0)), int(W.size(1)), int(W.size(0))
-    if x_rowmax is None:
-        x_rowmax = row_absmax(x)
-    _check_input(x_rowmax, "x_rowmax")
-    if x_rowmax.dim() != 2 or (x_rowmax.size(0) != 1 and x_rowmax.size(0) * rows_per_bound != rows):
-        raise RuntimeError("x_rowmax must be (rows / rows_per_bound, parts) or (1, parts)")
-    rowmax_stride = int(x_rowmax.size(1)) if x_rowmax.size(0) > 1 or rows == rows_per_bound else 0
-    if bias is not None:
-        _check_input(bias, "bias")
-        if bias.numel() != dim_out:
-            raise RuntimeError("bias size mismatch")
-    if rows % out_comps != 0:
-        raise RuntimeError("rows must be a multiple of out_comps")
-    y_shape = [rows, dim_out] if out_comps == 1 else [rows // out_comps, dim_out, out_comps]
-    with _on(x.device):
-        if out is None:
-            y = torch.empty(y_shape, dtype=torch.float32, device=x.device)
-        else:
-            _check_input(out, "out")
-            if out.numel() != rows * dim_out:
-                raise RuntimeError("out has wrong size")
-            y = out
-        ymax = None
-        if want_rowmax:
-            if out_comps != 1:
-                raise RuntimeError("row maxima are only produced for out_comps == 1")
-            parts = int(_lib.mg_tensor_linear_f16x2_rowmax_parts(rows, dim_in, dim_out))
-            ymax = torch.empty(rows, parts, dtype=torch.float32, device=x.device)
-        L.check(_lib.mg_tensor_linear_f16x2_scaled_bound(
-            _p(packed_weight_f16x2(W)), _p(x), _p(x_rowmax), int(x_rowmax.size(1)), rowmax_stride, int(rows_per_bound),
-            rows, dim_in, dim_out, _p(bias), int(act), int(bool(accumulate)), int(out_comps), _p(y), _p(ymax),
-            bound_mul, bound_add, _stream()))
+    y, ymax = _ext.linear_f16x2(W, x, *_bound_parts(x_rowmax), bias, act, out, accumulate, out_comps, want_rowmax,
+                                rows_per_bound, False)
     return (y, ymax) if want_rowmax else y
 
 
 LAYOUT_CHAN_COMP, LAYOUT_COMP_CHAN = 0, 1
+# rows x components from which a tensor linear goes through plain component rows and the split-fp16 kernels
+# (kComponentRows of csrc/torch_ops.cpp)
+COMPONENT_ROWS_MIN = 960
 
 
 def components_as_rows(inds, x):
@@ -1200,7 +1142,8 @@ def components_as_rows(inds, x):
     dim_in = int(x.size(x.dim() - 1 - inds))
     rows = x.numel() // (dim_in * T) if dim_in else 0
     k_pad = (dim_in + 31) // 32 * 32
-    if get_linear_mode() != LINEAR_F16X2 or rows * T < 32768 or k_pad > 256 or k_pad & (k_pad - 1):
+    if (get_linear_mode() != LINEAR_F16X2 or rows * T < COMPONENT_ROWS_MIN or dim_in <= 8 or k_pad > 256
+            or k_pad & (k_pad - 1)):
         return None
     with _on(x.device):
         x2 = torch.empty(rows * T, k_pad, dtype=torch.float32, device=x.device)
@@ -1211,7 +1154,7 @@ def components_as_rows(inds, x):
 
 def tensor_linear_fwd(inds, W, x, bias=None, act=ACT_NONE, out=None, accumulate=False,
                       x_layout=LAYOUT_CHAN_COMP, y_layout=LAYOUT_CHAN_COMP, row_bound=None, rows_per_bound=1,
-                      want_rowmax=False, x_rows=None):
+                      want_rowmax=False, x_rows=None, sequential=False):
     """y[..., o, t] = act(sum_i W[o, i] x[..., i, t] + bias[o]); W may have any strides.
     Layout 0 stores a tensor as (..., chan, (3,)^inds) like the reference; layout 1 is
     component-major (..., 3^inds, chan), the layout the fused edge kernels read and write.
@@ -1219,105 +1162,12 @@ def tensor_linear_fwd(inds, W, x, bias=None, act=ACT_NONE, out=None, accumulate=
     the kernel that produced x, used by the split-fp16 matrix path instead of a pass over x.
     want_rowmax: return (y, rowmax) with rowmax ((GEMM rows), parts) partial row maxima of |y| when the kernel
     that ran can emit them (plain-row output through the split-fp16 path), else (y, None).
-    x_rows: components_as_rows(inds, x) of this same x, if the caller has it (None is allowed)."""
-    if not W.is_cuda:
-        raise RuntimeError("W must be a CUDA tensor")
-    _check_input(x, "x")
-    if W.dtype != torch.float32:
-        raise RuntimeError("W must be float32")
-    if W.dim() != 2:
-        raise RuntimeError("expected W to be a matrix (2 dims)")
-    if inds > 2 or inds < 0:
-        raise RuntimeError("tensor_linear currently only supports a number of indices up to 2. "
-                           "go edit the code to add more (easy with copy/paste).")
-    dim_out, dim_in = int(W.size(0)), int(W.size(1))
-    T = 3 ** inds
-    if x_layout == LAYOUT_CHAN_COMP:
-        batch_dims = x.dim() - (1 + inds)
-        if batch_dims < 0:
-            raise RuntimeError("x has too few dims")
-        if x.size(batch_dims) != dim_in:
-            raise RuntimeError("channel dim size mismatch for x")
-        for i in range(batch_dims + 1, batch_dims + inds + 1):
-            if x.size(i) != 3:
-                raise RuntimeError("expected tensor index dim to be 3d for input x")
-    else:
-        batch_dims = x.dim() - 2
-        if batch_dims < 0 or x.size(-1) != dim_in or x.size(-2) != T:
-            raise RuntimeError("component-major x must have shape (..., 3^inds, dim_in)")
-    lead = [int(d) for d in x.shape[:batch_dims]]
-    rows = 1
-    for d in lead:
-        rows *= d
-    y_shape = lead + ([dim_out] + [3] * inds if y_layout == LAYOUT_CHAN_COMP else [T, dim_out])
-    if bias is not None:
-        _check_input(bias, "bias")
-        if bias.numel() != dim_out:
-            raise RuntimeError("bias size mismatch")
-    with _on(x.device):
-        if out is None:
-            y = torch.empty(y_shape, dtype=torch.float32, device=x.device)
-        else:
-            _check_input(out, "out")
-            if list(out.shape) != y_shape:
-                raise RuntimeError("out has wrong shape")
-            y = out
-        plain_rows = inds == 0 or x_layout == LAYOUT_COMP_CHAN
-        mode = get_linear_mode()
-        wide = (plain_rows and dim_in % 32 == 0 and dim_in >= 64 and dim_out >= 64 and rows * T >= 1024
-                and x.data_ptr() % 16 == 0)
-        out_comps = 1 if (inds == 0 or y_layout == LAYOUT_COMP_CHAN) else T
-        ymax = None
-
-        def rowmax_buffer(k_in):
-            if not (want_rowmax and out_comps == 1 and not accumulate):
-                return None
-            parts = int(_lib.mg_tensor_linear_f16x2_rowmax_parts(rows * T, k_in, dim_out))
-            return torch.empty(rows * T, parts, dtype=torch.float32, device=x.device)
-        if (mode == LINEAR_F16X2 and inds > 0 and x_layout == LAYOUT_CHAN_COMP and rows * T >= 32768 and dim_out >= 64
-                and row_bound is None and (y_layout == LAYOUT_COMP_CHAN or not (want_rowmax or accumulate or bias is not None
-                                                                                or act != ACT_NONE))):
-            # (row, chan, comp) -> (row, comp, chan) rows (K zero-padded to a multiple of 32), then the plain-row
-            # matrix path: its component-major output is written at the full store rate, which the generic
-            # kernel's layout mapping is not; with the reference's output layout its component epilogue still
-            # beats the generic kernel (61 against 104 us for 16384 x 128 x 3 -> 384)
-            k_pad = (dim_in + 31) // 32 * 32
-            if x_rows is not None and tuple(x_rows[0].shape) == (rows * T, k_pad):
-                x2, x2max = x_rows
-            elif k_pad <= 256 and k_pad & (k_pad - 1) == 0:
-                # transposition, padding and the row maxima in one pass
-                x2 = torch.empty(rows * T, k_pad, dtype=torch.float32, device=x.device)
-                x2max = torch.empty(rows * T, 1, dtype=torch.float32, device=x.device)
-                L.check(_lib.mg_components_to_rows(_p(x), rows, dim_in, T, k_pad, _p(x2), _p(x2max), _stream()))
-            else:
-                xt = x.reshape(rows, dim_in, T).transpose(1, 2)
-                xt = torch.nn.functional.pad(xt, (0, k_pad - dim_in)) if k_pad != dim_in else xt.contiguous()
-                x2 = xt.reshape(rows * T, k_pad)
-                x2max = row_absmax(x2)
-            Wp = zero_padded_columns(W, k_pad)
-            ymax = rowmax_buffer(k_pad)
-            L.check(_lib.mg_tensor_linear_f16x2(_p(packed_weight_f16x2(Wp)), _p(x2), _p(x2max), 1, 1, 1,
-                                                rows * T, k_pad, dim_out, _p(bias), int(act), int(bool(accumulate)),
-                                                out_comps, _p(y), _p(ymax), _stream()))
-        elif (plain_rows and mode == LINEAR_F16X2 and f16x2_supported(rows * T, dim_in, dim_out, x)):
-            x2 = x.reshape(rows * T, dim_in)
-            if row_bound is None:
-                row_bound, rows_per_bound = row_absmax(x2), 1
-            elif row_bound.dim() != 2 or row_bound.size(0) * rows_per_bound != rows * T:
-                raise RuntimeError("row_bound must be (rows / rows_per_bound, parts)")
-            ymax = rowmax_buffer(dim_in)
-            L.check(_lib.mg_tensor_linear_f16x2(_p(packed_weight_f16x2(W)), _p(x2), _p(row_bound),
-                                                int(row_bound.size(1)), int(row_bound.size(1)), int(rows_per_bound),
-                                                rows * T,
-                                                dim_in, dim_out, _p(bias), int(act), int(bool(accumulate)),
-                                                out_comps, _p(y), _p(ymax), _stream()))
-        elif wide and mode == LINEAR_BF16X3:
-            L.check(_lib.mg_tensor_linear_packed(_p(packed_weight(W)), _p(x), rows * T, dim_in, dim_out, _p(bias),
-                                                 int(act), int(bool(accumulate)), out_comps, _p(y), _stream()))
-        else:
-            L.check(_lib.mg_tensor_linear_layout(inds, _p(W), int(W.stride(0)), int(W.stride(1)), _p(x), rows,
-                                                 dim_in, dim_out, _p(bias), int(act), int(bool(accumulate)),
-                                                 int(x_layout), int(y_layout), _p(y), _stream()))
+    x_rows: components_as_rows(inds, x) of this same x, if the caller has it (None is allowed).
+    sequential: the reduction of an element runs over k in order whatever the number of rows is (few rows otherwise
+    split it over the waves of a workgroup)."""
+    x2, x2max = x_rows if x_rows is not None else (None, None)
+    y, ymax = _ext.linear_fwd(inds, W, x, bias, act, out, accumulate, x_layout, y_layout, *_bound_parts(row_bound),
+                              rows_per_bound, want_rowmax, x2, x2max, sequential)
     return (y, ymax) if want_rowmax else y
 
 
@@ -1327,62 +1177,7 @@ def tensor_linear_wgrad(inds, dy, x, dy_bound=None, x_bound=None, want_bias=Fals
     (float tensors of any shape whose largest magnitude bounds |dy| / |x|, e.g. row maxima that the caller already
     holds) save it a pass over the operand.  want_bias (inds = 0): returns (dW, db) with db[o] = sum over rows of
     dy[.., o], from the same pass where the kernel offers it."""
-    _check_input(dy, "dy")
-    _check_input(x, "x")
-    if want_bias and inds != 0:
-        raise RuntimeError("the bias gradient is defined for plain rows only")
-    batch_dims = x.dim() - (1 + inds)
-    dim_in, dim_out = int(x.size(batch_dims)), int(dy.size(batch_dims))
-    rows = 1
-    for i in range(batch_dims):
-        rows *= int(x.size(i))
-    with _on(x.device):
-        dW = torch.empty(dim_out, dim_in, dtype=torch.float32, device=x.device)
-        db = None
-        nbytes = ctypes.c_size_t(0)
-
-        def workspace(n_rows, n_in, n_out):
-            L.check(_lib.mg_tensor_linear_wgrad_workspace_bytes(n_rows, n_in, n_out, ctypes.byref(nbytes)))
-            return torch.empty(nbytes.value, dtype=torch.uint8, device=x.device)
-        if (inds == 0 and get_linear_mode() == LINEAR_F16X2 and x.data_ptr() % 16 == 0 and dy.data_ptr() % 16 == 0
-                and _lib.mg_tensor_linear_wgrad_f16x2_supported(rows, dim_in, dim_out)):
-            for b, name in ((dy_bound, "dy_bound"), (x_bound, "x_bound")):
-                if b is not None:
-                    _check_input(b, name)
-            if want_bias:
-                db = torch.empty(dim_out, dtype=torch.float32, device=x.device)
-            ws = workspace(rows, dim_in, dim_out)
-            L.check(_lib.mg_tensor_linear_wgrad_f16x2(
-                _p(dy), _p(x), _p(dy_bound), 0 if dy_bound is None else dy_bound.numel(),
-                _p(x_bound), 0 if x_bound is None else x_bound.numel(), rows, dim_in, dim_out, _p(ws), _p(dW), _p(db),
-                _stream()))
-        elif (inds > 0 and get_linear_mode() == LINEAR_F16X2 and rows * 3 ** inds >= 4096
-              and max(dim_in, dim_out) <= 256):
-            # (row, chan, comp) -> one plain row per (row, comp), channels zero-padded to a power of two: the sum over
-            # rows and components is then the plain-row weight gradient, on the matrix cores; the transposition
-            # also yields the row maxima the kernel scales by
-            T = 3 ** inds
-
-            def as_rows(t, dim):
-                pad = max(32, 1 << (dim - 1).bit_length())
-                out = torch.empty(rows * T, pad, dtype=torch.float32, device=t.device)
-                bound = torch.empty(rows * T, 1, dtype=torch.float32, device=t.device)
-                L.check(_lib.mg_components_to_rows(_p(t), rows, dim, T, pad, _p(out), _p(bound), _stream()))
-                return out, bound, pad
-            dy2, dy2_bound, o_pad = as_rows(dy, dim_out)
-            x2, x2_bound, i_pad = as_rows(x, dim_in)
-            ws = workspace(rows * T, i_pad, o_pad)
-            dW_pad = dW if (o_pad, i_pad) == (dim_out, dim_in) else torch.empty(o_pad, i_pad, dtype=torch.float32,
-                                                                                device=x.device)
-            L.check(_lib.mg_tensor_linear_wgrad_f16x2(_p(dy2), _p(x2), _p(dy2_bound), rows * T, _p(x2_bound), rows * T,
-                                                      rows * T, i_pad, o_pad, _p(ws), _p(dW_pad), None, _stream()))
-            if dW_pad is not dW:
-                dW = dW_pad[:dim_out, :dim_in].contiguous()
-        else:
-            ws = workspace(rows, dim_in, dim_out)
-            L.check(_lib.mg_tensor_linear_wgrad(inds, _p(dy), _p(x), rows, dim_in, dim_out, _p(ws), _p(dW), _stream()))
-            if want_bias:
-                db = dy.reshape(-1, dim_out).sum(0)
+    dW, db = _ext.linear_wgrad(inds, dy, x, dy_bound, x_bound, want_bias)
     return (dW, db) if want_bias else dW
 
 
@@ -2073,6 +1868,11 @@ def tensor_linear_f16x2_rowsum(W, x, x_bound, row_ptr, seg, n_out, bias=None, ac
         if bias.numel() != dim_out:
             raise RuntimeError("bias must have dim_out elements")
     dev = x.device
+    if rows and dim_out % 256 == 0 and _lib.mg_tensor_linear_f16x2_splits_k(rows, dim_in, dim_out):
+        # few rows: 256-row tiles would leave most of the chip idle
+        y = tensor_linear_f16x2(W, x, ScaledBound(x_bound, bound_mul, bound_add), bias=bias, act=act)
+        out = segment_sum_csr(y, row_ptr, n_out)
+        return (out if scale == 1.0 else out * scale), (y if want_rows else None)
     nbytes = ctypes.c_size_t(0)
     L.check(_lib.mg_tensor_linear_f16x2_rowsum_workspace_bytes(rows, dim_out, ctypes.byref(nbytes)))
     with _on(dev):

@@ -62,6 +62,16 @@ def _linear(x, lin, act, bound=None, want_bound=True):
     return y, ops.linear_out_bound(lin.weight, lin.bias, bound)
 
 
+_MLP_ACTS = (ops.ACT_SILU, ops.ACT_SILU, ops.ACT_NONE)
+
+
+def _mlp_params(mlp, last=None):
+    """([weights], [biases]) of an MLP's three linears; last: a layer to use in the last one's place."""
+    m = mlp.layers._modules
+    lins = (m["0"], m["2"], last if last is not None else m["4"])
+    return [lin.weight for lin in lins], [lin.bias for lin in lins]
+
+
 class MLP(nn.Module):
     """Linear, SiLU, Linear, SiLU, Linear (archs/meanflow_painn8.py:38-51); bias and
     activation are fused into the GEMM epilogue.  The wide layers run on the split-fp16 matrix
@@ -81,10 +91,9 @@ class MLP(nn.Module):
     def forward(self, x_a, bound=None):
         if diff.wants_grad(self, x_a):
             return diff.mlp_silu(self, x_a)
-        lead = x_a.shape[:-1]
         h = x_a.reshape(-1, x_a.shape[-1]).contiguous()
-        h, bound = _linear(h, self.layers[0], ops.ACT_SILU, bound)
-        return self.after_first(h, bound).reshape(*lead, -1)
+        y = ops.linear_chain(h, *_mlp_params(self), _MLP_ACTS, bound)
+        return y if x_a.dim() == 2 else y.reshape(*x_a.shape[:-1], -1)
 
     def hidden(self, x, bound=None):
         """The (rows, dim_out) input of the last layer and the bound of its rows."""
@@ -137,11 +146,6 @@ class Update(nn.Module):
         if diff.wants_grad(self, x_a, x_v):
             da, dv = diff.painn_update(self, x_a, x_v)
             return (diff.add(x_a, da), diff.add(x_v, dv)) if residual else (da, dv)
-        n = self.n
-        B, N = x_a.shape[:2]
-        rows = B * N
-        flat_a = x_a.reshape(rows, n).contiguous()
-        flat_v = x_v.reshape(rows, n, 3).contiguous()
         params = (self.lin_l.W, self.lin_r.W, self.lin_v.W)
         cache = self.__dict__.setdefault("_lrv_cache", {})
         stamp = ops.stamp(params)
@@ -149,15 +153,7 @@ class Update(nn.Module):
             with ops.derived_tensors():                                         # while the weights are unchanged, so
                 cache.update(stamp=stamp, W=torch.cat(params, dim=0))           # its packed planes stay valid too
         W = cache["W"]
-        # component-major (rows, 3, 3n): the GEMM stores whole rows, the two kernels below read with unit stride
-        lrv = ops.tensor_linear_fwd(1, W, flat_v, y_layout=ops.LAYOUT_COMP_CHAN)
-        ip, cat, cat_max = ops.painn_update_pre(lrv, flat_a, want_rowmax=True)  # l.r, [x_a | |r|] and its row maxima
-        y = self.mlp(cat, cat_max)                                              # (rows, 3n)
-        y3 = y.reshape(B, N, 3 * n)
-        out_a = self.gn(ip.reshape(B, N, n), mul=y3[..., n:2 * n], add=y3[..., 2 * n:],
-                        res=flat_a.reshape(B, N, n) if residual else None)
-        out_v = ops.painn_update_vec(lrv, y, flat_v if residual else None)
-        return out_a, out_v.reshape(B, N, n, 3)
+        return ops.painn_update(x_a.contiguous(), x_v.contiguous(), W, *_mlp_params(self.mlp), self.gn, residual)
 
 
 class Message(nn.Module):
@@ -190,6 +186,9 @@ class Message(nn.Module):
 
     use_sliced = True
     use_cell_order = True
+    # Edges from which the filter MLP's last layers run inside the edge kernel.  Its tiles are 256 edges x 256 columns: 6000
+    # edges are 47 workgroups and take 61 us, a stored filter from GEMMs cut to the problem and the plain edge kernel 25.
+    FOLD_EDGES = 32768
 
     def _sliced_actv_last(self):
         """Last layer of mlp_actv with its rows in the slice-major column order of painn_table_message_sliced."""
@@ -264,18 +263,18 @@ class Message(nn.Module):
         return kept[1]
 
     def _evaluate_filter_table(self, rows, shift=0.0):
-        first = self.mlp_dist.layers[0]
-        device = first.weight.device
-        unit = ops.linear_in_unit_bound(device)
-        if (self.n_rbf < self.GRID_K and ops.get_linear_mode() == ops.LINEAR_F16X2 and not diff.wants_grad(self.mlp_dist)
-                and ops.f16x2_supported(rows, self.GRID_K, first.out_features, first.weight)):
-            # a reduction dimension of n_rbf is below what the matrix path takes: the encodings (constants of the
-            # grid) and the weight's columns are padded with zeros, which leaves every product as it was
-            enc = self._grid_encoding(rows, shift, device, self.GRID_K)
-            h = ops.tensor_linear_f16x2(ops.zero_padded_columns(first.weight, self.GRID_K), enc, unit,
-                                        bias=first.bias, act=ops.ACT_SILU)
-            return self.mlp_dist.after_first(h, ops.linear_out_bound(first.weight, first.bias, unit))
-        return self.mlp_dist(self._grid_encoding(rows, shift, device), unit)
+        if diff.wants_grad(self.mlp_dist):
+            return self.mlp_dist(self._grid_encoding(rows, shift, self.mlp_dist.layers[0].weight.device))
+        return ops.filter_grid(*self._grid_inputs(rows, shift))
+
+    def _grid_inputs(self, rows, shift=0.0):
+        """(encodings of the grid, a unit bound of them, weights, biases) for ops.filter_grid.  A reduction dimension of n_rbf below
+        GRID_K is less than what the matrix path takes: the encodings (constants of the grid) and the weight's columns
+        are then padded with zeros, which leaves every product as it was."""
+        W, b = _mlp_params(self.mlp_dist)
+        device = W[0].device
+        pad = self.n_rbf < self.GRID_K and ops.get_linear_mode() == ops.LINEAR_F16X2 and W[0].shape[0] >= 8
+        return (self._grid_encoding(rows, shift, device, self.GRID_K if pad else None), ops.linear_in_unit_bound(device), W, b)
 
     def _grid_phases(self, rows, shift):
         """The float64 encodings at d = (k + shift) 2 r0 / rows (host tensor)."""
@@ -338,54 +337,44 @@ class Message(nn.Module):
             da, dv = diff.painn_message(self, graph, x_a, x_v, r_ij)
             return (diff.add(x_a, da), diff.add(x_v, dv)) if residual else (da, dv)
         B, N, n = x_a.shape
-        flat_a = x_a.reshape(B * N, n).contiguous()
-        flat_v = x_v.reshape(B * N, n, 3).contiguous()
-        r_ij = r_ij.contiguous()
-        res_a, res_v = (flat_a, flat_v) if residual else (None, None)
-        actv = None
-        if self.use_table and n % 4 == 0 and r_ij.shape[0] >= 4 * self.TABLE_ROWS[0]:
+        x_a, x_v, r_ij = x_a.contiguous(), x_v.contiguous(), r_ij.contiguous()
+        E = r_ij.shape[0]
+        if self.use_table and n % 4 == 0 and E >= 4 * self.TABLE_ROWS[0]:
             rows = self.table_rows()
-            if rows and rows <= ops.PAINN_SLICED_MAX_ROWS and n % ops.PAINN_SLICE == 0 and self.use_sliced:
-                # the grid fits in LDS: actv comes out of its MLP with the columns regrouped slice by slice
-                h_a, b_a = self.mlp_actv.hidden(flat_a)
-                actv_s = _linear(h_a, self._sliced_actv_last(), ops.ACT_NONE, b_a, want_bound=False)[0]
-                # rows in cell order when the graph has one: consecutive rows then gather the same neighbours
-                order = getattr(graph, "cell_order", None) if self.use_cell_order else None
-                out_a, out_v = ops.painn_table_message_sliced(graph.row_ptr, graph.dst32, r_ij, self.filter_table(rows),
-                                                              2.0 * self.r0, actv_s, flat_v, self.epsilon, res_a, res_v,
-                                                              node_order=order)
-                return out_a.reshape(B, N, n), out_v.reshape(B, N, n, 3)
-            actv = self.mlp_actv(flat_a)
-            if rows and r_ij.shape[0] >= 4 * rows:
-                # the grid is re-evaluated in every call (a few thousand rows): nothing of a forward is cached
-                out_a, out_v = ops.painn_table_message(graph.row_ptr, graph.dst32, r_ij, self.filter_table(rows),
-                                                       2.0 * self.r0, actv, flat_v, self.epsilon, res_a, res_v)
-                return out_a.reshape(B, N, n), out_v.reshape(B, N, n, 3)
+            sliced = rows and rows <= ops.PAINN_SLICED_MAX_ROWS and n % ops.PAINN_SLICE == 0 and self.use_sliced
+            if sliced or (rows and E >= 4 * rows):
+                # The grid is re-evaluated in every call (a few thousand rows): nothing of a forward is cached.  Where it
+                # fits in LDS, actv comes out of its MLP with the columns regrouped slice by slice, and the rows are taken
+                # in cell order when the graph has one: consecutive rows then gather the same neighbours.
+                order = getattr(graph, "cell_order", None) if sliced and self.use_cell_order else None
+                table = self.filter_table(rows) if self.keep_table else None
+                return ops.painn_message_grid(graph.row_ptr, graph.dst32, r_ij, order, x_a, x_v,
+                                              *_mlp_params(self.mlp_actv, self._sliced_actv_last() if sliced else None),
+                                              *self._grid_inputs(rows), table, 2.0 * self.r0, self.epsilon, sliced, residual)
         if getattr(graph, "padded", False):
             # the edge arrays are longer than the graph: only the kernels above, which reach the edges through
             # row_ptr, are valid; the per-edge GEMMs below would also process the rows past the edge count
             raise RuntimeError("Message.forward on a capacity-sized graph needs the filter-grid path "
                                "(n a multiple of 16, a grid accepted for these weights, edge capacity >= 4 x grid rows)")
-        if actv is None:
-            actv = self.mlp_actv(flat_a)
-        if ops.painn_filter_message_supported(n, 4 * n, r_ij.shape[0]):
-            # the filter's last layer runs inside the edge kernel: the (edges, 4n) filter is never stored
-            first, second = self.mlp_dist.layers[0], self.mlp_dist.layers[2]
-            if ops.painn_filter_hidden_supported(self.n_rbf, second.out_features, r_ij.shape[0]):
-                # encoding, first and second layer in one kernel: the first layer's output is never stored
-                b1 = ops.linear_out_bound(first.weight, first.bias, None)
-                h = ops.painn_filter_hidden(r_ij, self.r0, first.weight, first.bias, second.weight, second.bias, b1)
-                bound = ops.linear_out_bound(second.weight, second.bias, b1)
-            else:
-                h, bound = self._hidden(r_ij)
-                h, bound = _linear(h, second, ops.ACT_SILU, bound)
-            W3, b3 = self._permuted_last()
-            out_a, out_v = ops.painn_filter_message(W3, b3, h, bound, graph.row_ptr, graph.src32, graph.dst32, r_ij,
-                                                    actv, flat_v, self.epsilon, res_a, res_v)
-            return out_a.reshape(B, N, n), out_v.reshape(B, N, n, 3)
-        filt = self.filters(r_ij)
-        out_a, out_v = ops.painn_message(graph.row_ptr, graph.dst32, r_ij, filt, actv, flat_v,
-                                         self.epsilon, res_a, res_v)
+        if E < self.FOLD_EDGES or not ops.painn_filter_message_supported(n, 4 * n, E):
+            return ops.painn_message_edges(graph.row_ptr, graph.dst32, r_ij, x_a, x_v, *_mlp_params(self.mlp_actv),
+                                           *_mlp_params(self.mlp_dist), self.r0, self.epsilon, residual)
+        flat_a, flat_v = x_a.reshape(B * N, n), x_v.reshape(B * N, n, 3)
+        res_a, res_v = (flat_a, flat_v) if residual else (None, None)
+        actv = self.mlp_actv(flat_a)
+        # the filter's last layer runs inside the edge kernel: the (edges, 4n) filter is never stored
+        first, second = self.mlp_dist.layers[0], self.mlp_dist.layers[2]
+        if ops.painn_filter_hidden_supported(self.n_rbf, second.out_features, E):
+            # encoding, first and second layer in one kernel: the first layer's output is never stored
+            b1 = ops.linear_out_bound(first.weight, first.bias, None)
+            h = ops.painn_filter_hidden(r_ij, self.r0, first.weight, first.bias, second.weight, second.bias, b1)
+            bound = ops.linear_out_bound(second.weight, second.bias, b1)
+        else:
+            h, bound = self._hidden(r_ij)
+            h, bound = _linear(h, second, ops.ACT_SILU, bound)
+        W3, b3 = self._permuted_last()
+        out_a, out_v = ops.painn_filter_message(W3, b3, h, bound, graph.row_ptr, graph.src32, graph.dst32, r_ij,
+                                                actv, flat_v, self.epsilon, res_a, res_v)
         return out_a.reshape(B, N, n), out_v.reshape(B, N, n, 3)
 
 

@@ -25,10 +25,14 @@ class _TensorLinearFn(torch.autograd.Function):
     number of times, as torch.autograd.functional.jvp(create_graph=True) of the meanflow loss needs
     (archs/meanflow_painn8.py:274-282); the reference's C++ backward calls raw kernels and cannot.
     x_bound: row maxima of |x| when the caller already holds them (a scaling hint, not differentiated).
-    bias (plain rows only): added in the kernel's epilogue; its gradient comes out of the weight-gradient pass."""
+    bias (plain rows only): added in the kernel's epilogue; its gradient comes out of the weight-gradient pass.
+    sequential: every element's reduction in k order whatever the number of rows (ops.tensor_linear_fwd).  The layers that
+    lead to a LeakyReLU ask for it in their forward pass: the derivative jumps at zero, so a pre-activation within rounding
+    of zero takes one slope or the other, and a row's gradient must not depend on the size of the batch around it.
+    Gradients, and networks of smooth activations, take the faster split reduction."""
 
     @staticmethod
-    def forward(ctx, inds, W, x, x_bound=None, bias=None, want_bound=False):
+    def forward(ctx, inds, W, x, x_bound=None, bias=None, want_bound=False, sequential=False):
         ctx.inds = inds
         x = x.contiguous()
         if x_bound is None:
@@ -41,9 +45,9 @@ class _TensorLinearFn(torch.autograd.Function):
         ctx.set_materialize_grads(False)
         bias = None if bias is None else bias.contiguous()
         if not want_bound:
-            return ops.tensor_linear_fwd(inds, W, x, bias=bias, row_bound=x_bound)
+            return ops.tensor_linear_fwd(inds, W, x, bias=bias, row_bound=x_bound, sequential=sequential)
         # the kernel's partial row maxima of |y| (an empty tensor when the kernel that ran does not produce them)
-        y, y_bound = ops.tensor_linear_fwd(inds, W, x, bias=bias, row_bound=x_bound, want_rowmax=True)
+        y, y_bound = ops.tensor_linear_fwd(inds, W, x, bias=bias, row_bound=x_bound, want_rowmax=True, sequential=sequential)
         if y_bound is None:
             y_bound = y.new_empty(0)
         ctx.mark_non_differentiable(y_bound)
@@ -69,7 +73,7 @@ class _TensorLinearFn(torch.autograd.Function):
     def backward(ctx, dy, *_):
         W, x = ctx.saved_tensors
         if dy is None:
-            return None, None, None, None, None, None
+            return None, None, None, None, None, None, None
         dy = dy.contiguous()
         dW = dx = db = None
         dy_bound = _row_bound(ctx.inds, dy)
@@ -80,7 +84,7 @@ class _TensorLinearFn(torch.autograd.Function):
                 db = None
         if ctx.needs_input_grad[2]:
             dx = _TensorLinearFn.apply(ctx.inds, W.t(), dy, dy_bound)   # strides of W are honoured: no copy
-        return None, dW, dx, None, db, None
+        return None, dW, dx, None, db, None, None
 
 
 class _WeightGradFn(torch.autograd.Function):
@@ -115,7 +119,7 @@ class _WeightGradFn(torch.autograd.Function):
         return None, g_dy, g_x, None, None, None
 
 
-def tensor_linear(inds, W, x, bias=None, x_bound=None, want_bound=False):
+def tensor_linear(inds, W, x, bias=None, x_bound=None, want_bound=False, sequential=False):
     """bias (inds = 0 only): y = x W^T + bias in one kernel.  x_bound: upper bounds of the row maxima of |x|
     ((rows, parts)) when the caller holds them.  want_bound: returns (y, bound) with the kernel's partial row maxima
     of |y|, or None where the kernel that ran does not produce them: they bound |f(y)| for any f with |f(z)| <= |z|
@@ -124,8 +128,8 @@ def tensor_linear(inds, W, x, bias=None, x_bound=None, want_bound=False):
         raise RuntimeError("a bias is defined for plain rows only")
     x = x.contiguous()          # (here, where autograd records the copy: the function saves x for later derivatives)
     if not want_bound:
-        return _TensorLinearFn.apply(inds, W, x, x_bound, bias)
-    y, y_bound = _TensorLinearFn.apply(inds, W, x, x_bound, bias, True)
+        return _TensorLinearFn.apply(inds, W, x, x_bound, bias, False, sequential)
+    y, y_bound = _TensorLinearFn.apply(inds, W, x, x_bound, bias, True, sequential)
     return y, (y_bound if y_bound.numel() else None)
 
 
@@ -143,7 +147,7 @@ class TensLinear(nn.Module):
         nn.init.normal_(self.W, std=fan_in ** -0.5)
 
     def forward(self, x):
-        return tensor_linear(self.inds, self.W, x.contiguous())
+        return tensor_linear(self.inds, self.W, x.contiguous(), sequential=torch.is_grad_enabled())
 
 
 class TensorProdBare(nn.Module):

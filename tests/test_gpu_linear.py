@@ -558,3 +558,46 @@ def test_weight_gradient_at_the_edge_count_of_configs2(ops):
     assert float((got_b.double() - want_b).abs().max()) <= 1e-6 + 1e-5 * float(want_b.abs().max())
     again, again_b = ops.tensor_linear_wgrad(0, dy, x, want_bias=True)
     assert torch.equal(again, got) and torch.equal(again_b, got_b)
+
+
+# around the crossovers of the split-K kernel (256 / 512 / 1536 blocks of 32 x 32, four and eight waves, partial row and
+# column blocks) and one problem past them; dim_in 96 leaves one of its four waves without a chunk
+@pytest.mark.parametrize("rows,dim_in,dim_out", [(1, 512, 512), (31, 64, 40), (33, 96, 512), (512, 256, 512), (544, 256, 512),
+                                                 (1025, 512, 512), (3072, 512, 512), (3105, 512, 512), (6145, 1280, 64),
+                                                 (700, 768, 100)])
+@pytest.mark.parametrize("act", [0, 1, 2])
+def test_linear_f16x2_split_reduction(ops, rows, dim_in, dim_out, act):
+    """Few rows: the reduction split over the waves of a workgroup, with the row maxima it emits; sequential=True gives every
+    row the bits it has in a batch too large to split."""
+    g = torch.Generator().manual_seed(rows + dim_in)
+    x = (torch.randn(rows, dim_in, generator=g) * (torch.rand(rows, 1, generator=g) * 3)).cuda()
+    W = (torch.randn(dim_out, dim_in, generator=g) / dim_in ** 0.5).cuda()
+    b = torch.randn(dim_out, generator=g).cuda()
+    y, ymax = ops.tensor_linear_f16x2(W, x, ops.row_absmax(x), bias=b, act=act, want_rowmax=True)
+
+    def ref(dt):
+        z = x.cpu().to(dt) @ W.cpu().to(dt).T + b.cpu().to(dt)
+        return torch.nn.functional.silu(z) if act == 1 else (torch.nn.functional.leaky_relu(z, 0.1) if act == 2 else z)
+    _check(y, ref, f"split reduction {rows} x {dim_in} -> {dim_out}")
+    assert torch.equal(ymax.amax(1), y.abs().amax(1))
+    if rows >= 256:
+        many = x.repeat(60, 1)[:60000]
+        a = ops.tensor_linear_fwd(0, W, x, bias=b, act=act, sequential=True)
+        assert torch.equal(a, ops.tensor_linear_fwd(0, W, many, bias=b, act=act)[:rows])
+
+
+@pytest.mark.parametrize("inds,dim_in", [(0, 1), (0, 8), (0, 20), (0, 32), (1, 1), (1, 8), (2, 3)])
+@pytest.mark.parametrize("rows,dim_out", [(1, 5), (63, 256), (700, 300)])
+def test_linear_few_inputs(ops, inds, dim_in, rows, dim_out):
+    g = torch.Generator().manual_seed(rows + dim_in)
+    x = torch.randn(rows, dim_in, *([3] * inds), generator=g)
+    W, b = torch.randn(dim_out, dim_in, generator=g), torch.randn(dim_out, generator=g)
+    T = 3 ** inds
+    y = ops.tensor_linear_fwd(inds, W.cuda(), x.cuda())
+    _check(y, lambda dt: OP.tensor_linear(inds, W.to(dt), x.to(dt)), "few inputs")
+    if inds == 0:
+        y2 = ops.tensor_linear_fwd(0, W.cuda(), x.cuda(), bias=b.cuda(), act=ops.ACT_SILU, out=y.clone(), accumulate=True)
+        _check(y2, lambda dt: y.cpu().to(dt) + torch.nn.functional.silu(x.to(dt) @ W.to(dt).T + b.to(dt)), "few inputs, accumulated")
+    else:
+        y2 = ops.tensor_linear_fwd(inds, W.cuda(), x.cuda(), y_layout=ops.LAYOUT_COMP_CHAN)
+        assert torch.equal(y2.reshape(rows, T, dim_out).transpose(1, 2), y.reshape(rows, dim_out, T))
