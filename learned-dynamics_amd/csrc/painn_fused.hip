@@ -121,6 +121,7 @@ __device__ __forceinline__ void wfirst_gemm_tile(floatx16 (&acc)[kFNI], const _F
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bl, ah[s], acc[ni], 0, 0, 0);
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bh, ah[s], acc[ni], 0, 0, 0);
             }
+        order_chunk<kFNI>();
     };
 
     unsigned char* buf0 = lds;

@@ -268,6 +268,7 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s], bl, acc[ni], 0, 0, 0);
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s], bh, acc[ni], 0, 0, 0);
             }
+        order_chunk<NI>();
     };
 
     unsigned char* buf0 = lds;
