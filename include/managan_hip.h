@@ -320,6 +320,14 @@ int mg_linear_f16x2_pack_weight(const float* W, long w_stride_o, long w_stride_i
 /* the same with zero columns appended up to dim_pad (a multiple of 32): the packed weight of a reduction that long */
 int mg_linear_f16x2_pack_weight_padded(const float* W, long w_stride_o, long w_stride_i, int dim_in, int dim_out, int dim_pad,
                                        void* packed, mg_stream_t stream);
+/* and several weights in one launch */
+typedef struct mg_f16x2_weight {
+    const float* W;              /* element (o, i) at o stride_o + i stride_i */
+    long stride_o, stride_i;
+    int dim_in, dim_out, dim_pad;
+    void* packed;                /* mg_linear_f16x2_packed_weight_bytes(dim_pad, dim_out) bytes, 16-byte aligned */
+} mg_f16x2_weight;
+int mg_linear_f16x2_pack_weights(const mg_f16x2_weight* weights /* host */, int count, mg_stream_t stream);
 int mg_row_absmax(const float* x, long rows, int dim, float* out /* (rows) */, mg_stream_t stream);
 int mg_tensor_linear_f16x2_rowmax_parts(long rows, int dim_in, int dim_out);
 /* 1 when mg_tensor_linear_f16x2 splits the reduction of a problem of this size over the waves of a workgroup (few rows)
@@ -382,6 +390,10 @@ int mg_tensor_linear_wgrad_f16x2_supported(long rows, int dim_in, int dim_out); 
 int mg_tensor_linear_wgrad_f16x2(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,
                                  const float* x_bound, long n_x_bound, long rows, int dim_in, int dim_out,
                                  void* workspace, float* dW, float* db /* (dim_out) or NULL */, mg_stream_t stream);
+/* the same with db summed over the first bias_rows rows only (rows of values before rows of their tangents) */
+int mg_tensor_linear_wgrad_f16x2_rows(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,
+                                      const float* x_bound, long n_x_bound, long rows, long bias_rows, int dim_in, int dim_out,
+                                      void* workspace, float* dW, float* db /* (dim_out) or NULL */, mg_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Ant16 (managan/codegen_tensor_products.py:19-34; ant16_o0_cuda / ant16_o1_cuda / ant16_o2_cuda /
@@ -556,6 +568,56 @@ int mg_bee_edge_filters_bwd(const float* enc, const float* rh, const float* g_v,
  * to three times by the meanflow loss, :274-296): out[k] = SiLU^(order)(z[k]) (* mul[k] if mul is not null), order 0..4,
  * n floats, 16-byte aligned.  The reference leaves these derivatives to autograd's elementwise formulas. */
 int mg_silu_order(const float* z, const float* mul, long n, int order, float* out, mg_stream_t stream);
+
+/* The PaiNN layers under differentiation (archs/meanflow_painn8.py:25-100; the meanflow loss, :274-296): the passes between the
+ * linear maps, forward and adjoint.  dual != 0: every array holds `rows` rows of values and then `rows` rows of forward-mode
+ * tangents, and both halves are read and written in one pass; dual == 0: values alone.  n is a multiple of 4, arrays of rows are
+ * 16-byte aligned.  *_rowmax: upper bounds of the row maxima of what was written, which the linears scale by.
+ *
+ * The activation of a layer: h = SiLU(z), h_t = SiLU'(z) z_t, and its adjoint. */
+int mg_silu_rows_fwd(const float* z, long rows, int n, int dual, float* h, mg_stream_t stream);
+int mg_silu_rows_bwd(const float* z, const float* dh, long rows, int n, int dual, float* dz, float* dz_rowmax, mg_stream_t stream);
+/* Edge vectors r (E, 3) [and tangents r_t] -> enc = radial_encode(r, n, rmax) ((1 or 2) E, n) and dir = r / sqrt(|r|^2 + eps)
+ * [and dir_t]; the adjoint gives g_r [and g_r_t].  r_t == NULL: values alone. */
+int mg_painn_edge_encode_fwd(const float* r, const float* r_t, long E, int n, float rmax, float eps, float* enc, float* enc_rowmax,
+                             float* dir, float* dir_t, mg_stream_t stream);
+int mg_painn_edge_encode_bwd(const float* r, const float* r_t, long E, int n, float rmax, float eps, const float* g_enc,
+                             const float* g_dir, const float* g_dir_t, float* g_r, float* g_r_t, mg_stream_t stream);
+/* The message (archs/meanflow_painn8.py:94-100) and its tangent: dist (E, 4n) and dir (E, 3) per edge, actv (n_rows, 4n) and
+ * v (n_rows, n, 3) per node, read at node[e]; sums over the edges row_ptr[r] .. row_ptr[r + 1] - 1 of an output row.  A tangent
+ * that is NULL is zero. */
+typedef struct mg_painn_combine_dual {
+    const float *dist, *dist_t, *actv, *actv_t, *v, *v_t, *dir, *dir_t;
+    long E, n_rows;
+    int n;                       /* a power of two in 4..256 */
+} mg_painn_combine_dual;
+int mg_painn_combine_dual_fwd(const mg_painn_combine_dual* in, const int* node, const int* row_ptr, long n_out, float* out_v,
+                              float* out_v_t, float* out_a, float* out_a_t, mg_stream_t stream);
+/* Its adjoint: g_v, g_a, g_v_t, g_a_t are read at grad_row[e]; row_ptr / order list the edges that read a row of actv and v
+ * (order == NULL: the positions themselves).  A gradient that is NULL is not wanted. */
+typedef struct mg_painn_combine_dual_grad {
+    float *dist, *dist_t, *actv, *actv_t, *v, *v_t, *dir, *dir_t;
+} mg_painn_combine_dual_grad;
+int mg_painn_combine_dual_bwd(const mg_painn_combine_dual* in, const int* row_ptr, const int* order, const float* g_v,
+                              const float* g_v_t, const float* g_a, const float* g_a_t, const int* grad_row, long n_grad_rows,
+                              const mg_painn_combine_dual_grad* grad, mg_stream_t stream);
+/* The update (archs/meanflow_painn8.py:63-75) around its MLP.  lrv (rows, 3, 3n): the maps l, r, v of x_v, component-major.
+ * pre: ip = l . r, cat = [x_a, |r|].  post, with y = mlp(cat) (rows, 3n) and rows = batch x nodes:
+ * out_a = groupnorm(ip y2) + y3, out_v = w / sqrt(|w|^2 + 1), w = v y1.  stats: 4 floats per box and group, written by post_fwd
+ * and read by post_bwd.  post_bwd writes g_y, g_ip, the v third of g_lrv and the gradients of gamma and beta; pre_bwd the other
+ * two thirds and g_xa. */
+int mg_painn_update_pre_fwd(const float* lrv, const float* x_a, const float* x_a_t, long rows, int n, int dual, float* ip,
+                            float* cat, float* cat_rowmax, mg_stream_t stream);
+int mg_painn_update_scratch_floats(int batch, int nodes, int n, int groups, long* forward, long* backward /* host */);
+int mg_painn_update_post_fwd(const float* lrv, const float* ip, const float* y, const float* gamma, const float* beta, int batch,
+                             int nodes, int n, int groups, float eps, int dual, float* scratch, float* stats, float* out_a,
+                             float* out_v, mg_stream_t stream);
+int mg_painn_update_post_bwd(const float* lrv, const float* ip, const float* y, const float* stats, const float* gamma,
+                             const float* g_a, const float* g_a_t, const float* g_v, const float* g_v_t, int batch, int nodes, int n,
+                             int groups, int dual, float* scratch, float* g_y, float* g_y_rowmax, float* g_ip, float* g_lrv,
+                             float* d_gamma, float* d_beta, mg_stream_t stream);
+int mg_painn_update_pre_bwd(const float* lrv, const float* g_ip, const float* g_cat, long rows, int n, int dual, float* g_lrv,
+                            float* g_lrv_rowmax, float* g_xa, mg_stream_t stream);
 
 /* The first two layers of the radial MLP from the edge vectors (archs/meanflow_painn8.py:25-35 feeding :38-51):
  *   y[e] = SiLU(b2 + W2 SiLU(b1 + W1 radial_encode(r_ij[e], 16, rmax))),   y (E, hidden)

@@ -62,6 +62,7 @@ _SIGNATURES = {
     "mg_tensor_linear_wgrad_workspace_bytes": [i64, i32, i32, ctypes.POINTER(ctypes.c_size_t)],
     "mg_tensor_linear_wgrad": [i32, vp, vp, i64, i32, i32, vp, vp, vp],
     "mg_tensor_linear_wgrad_f16x2_supported": [i64, i32, i32],
+    "mg_tensor_linear_wgrad_f16x2_rows": [vp, vp, vp, i64, vp, i64, i64, i64, i32, i32, vp, vp, vp, vp],
     "mg_tensor_linear_wgrad_f16x2": [vp, vp, vp, i64, vp, i64, i64, i32, i32, vp, vp, vp, vp],
     "mg_tensor_linear_layout": [i32, vp, i64, i64, vp, i64, i32, i32, vp, i32, i32, i32, i32, vp, vp],
     "mg_bee_edge_geometry": [vp, i64, f32, vp, vp, vp],
@@ -81,6 +82,7 @@ _SIGNATURES = {
     "mg_tensor_linear_f16x2_run": [vp, vp],
     "mg_tensor_linear_f16x2_rowmax_parts_sequential": [i64, i32, i32],
     "mg_linear_f16x2_pack_weight_padded": [vp, i64, i64, i32, i32, i32, vp, vp],
+    "mg_linear_f16x2_pack_weights": [vp, i32, vp],
     "mg_tensor_linear_f16x2_splits_k": [i64, i32, i32],
     "mg_tensor_linear_f16x2_rowmax_parts": [i64, i32, i32],
     "mg_tensor_linear_f16x2": [vp, vp, vp, i32, i64, i64, i64, i32, i32, vp, i32, i32, i32, vp, vp, vp],
@@ -113,6 +115,17 @@ _SIGNATURES = {
     "mg_painn_table_message_sliced": [vp, vp, vp, i32, i64, vp, vp, i32, vp, vp, i32, vp, vp, vp, vp, vp],
     "mg_painn_combine_supported": [i32],
     "mg_silu_order": [vp, vp, i64, i32, vp, vp],
+    "mg_silu_rows_fwd": [vp, i64, i32, i32, vp, vp],
+    "mg_silu_rows_bwd": [vp, vp, i64, i32, i32, vp, vp, vp],
+    "mg_painn_edge_encode_fwd": [vp, vp, i64, i32, f32, f32, vp, vp, vp, vp, vp],
+    "mg_painn_edge_encode_bwd": [vp, vp, i64, i32, f32, f32, vp, vp, vp, vp, vp, vp],
+    "mg_painn_combine_dual_fwd": [vp, vp, vp, i64, vp, vp, vp, vp, vp],
+    "mg_painn_combine_dual_bwd": [vp, vp, vp, vp, vp, vp, vp, vp, i64, vp, vp],
+    "mg_painn_update_pre_fwd": [vp, vp, vp, i64, i32, i32, vp, vp, vp, vp],
+    "mg_painn_update_scratch_floats": [i32, i32, i32, i32, vp, vp],
+    "mg_painn_update_post_fwd": [vp, vp, vp, vp, vp, i32, i32, i32, i32, f32, i32, vp, vp, vp, vp, vp],
+    "mg_painn_update_post_bwd": [vp, vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, vp, vp, vp, vp, vp, vp, vp, vp],
+    "mg_painn_update_pre_bwd": [vp, vp, vp, i64, i32, i32, vp, vp, vp, vp],
     "mg_bee_edge_filters_fwd": [vp, vp, i64, i32, vp, vp, vp],
     "mg_bee_edge_filters_bwd": [vp, vp, vp, vp, i64, i32, vp, vp, vp],
     "mg_painn_table_interp_supported": [i32, i32],

@@ -59,12 +59,30 @@ __device__ __forceinline__ float activate_c(float v) {
 // of |w|: any order gives the same) and the split.  One pass over W for I <= kPackRegs * 256.  I_w <= I: columns of W, the
 // others are zeros.
 constexpr int kPackThreads = 1024, kPackRegs = 4;
-__global__ void __launch_bounds__(kPackThreads) pack_weight_f16x2_kernel(const float* __restrict__ W, long so, long si, int I_w,
-                                                                         int I, int O, int O_pad, _Float16* __restrict__ planes,
-                                                                         float* __restrict__ inv_scale) {
+// A launch takes up to kPackJobs weights (a training step packs every weight of a layer and its transpose anew: one launch of
+// 10 us per MLP instead of six of 6).
+constexpr int kPackJobs = 8;
+struct PackJob {
+    const float* W;
+    long so, si;
+    int I_w, I, O, O_pad, first_block;
+    _Float16* planes;
+};
+struct PackJobs {
+    PackJob job[kPackJobs];
+    int count;
+};
+__global__ void __launch_bounds__(kPackThreads) pack_weight_f16x2_kernel(const PackJobs jobs) {
     __shared__ unsigned row_max[32];
     const int tid = threadIdx.x;
-    const int block = blockIdx.x;
+    int which = 0;
+    while (which + 1 < jobs.count && (int)blockIdx.x >= jobs.job[which + 1].first_block) which++;     // (uniform)
+    const PackJob& job = jobs.job[which];
+    const float* __restrict__ W = job.W;
+    const long so = job.so, si = job.si;
+    const int I_w = job.I_w, I = job.I, O = job.O, O_pad = job.O_pad, block = blockIdx.x - job.first_block;
+    _Float16* __restrict__ planes = job.planes;
+    float* __restrict__ inv_scale = reinterpret_cast<float*>(planes + 2L * O_pad * I);
     const int m = tid & 31;
     const long o = 32L * block + m;
     const int pieces = I >> 3;                            // per row; thread t takes pieces t / 32, + 32, ...
@@ -629,18 +647,38 @@ int mg_linear_f16x2_packed_weight_bytes(int dim_in, int dim_out, size_t* bytes) 
     return MG_OK;
 }
 
+int mg_linear_f16x2_pack_weights(const mg_f16x2_weight* weights, int count, mg_stream_t stream) {
+    MG_REQUIRE(count >= 0 && (weights || count == 0), "mg_linear_f16x2_pack_weights: bad argument");
+    PackJobs jobs;
+    int blocks = 0;
+    jobs.count = 0;
+    auto flush = [&]() -> int {
+        if (jobs.count == 0) return MG_OK;
+        hipLaunchKernelGGL(pack_weight_f16x2_kernel, dim3((unsigned)blocks), dim3(kPackThreads), 0, (hipStream_t)stream, jobs);
+        blocks = 0;
+        jobs.count = 0;
+        return check_launch("mg_linear_f16x2_pack_weight");
+    };
+    for (int k = 0; k < count; k++) {
+        const mg_f16x2_weight& w = weights[k];
+        MG_REQUIRE(w.dim_in >= 0 && w.dim_out >= 0 && w.dim_pad >= w.dim_in, "mg_linear_f16x2_pack_weight: bad size");
+        if (w.dim_in == 0 || w.dim_out == 0) continue;
+        MG_REQUIRE(w.W && w.packed && aligned16(w.packed), "mg_linear_f16x2_pack_weight: null or unaligned pointer");
+        MG_REQUIRE(w.dim_pad % 32 == 0, "mg_linear_f16x2_pack_weight: dim_in must be a multiple of 32");
+        const int O_pad = o_pad_of(w.dim_out);
+        jobs.job[jobs.count++] = PackJob{w.W, w.stride_o, w.stride_i, w.dim_in, w.dim_pad, w.dim_out, O_pad, blocks,
+                                         static_cast<_Float16*>(w.packed)};
+        blocks += O_pad / 32;
+        if (jobs.count == kPackJobs)
+            if (int code = flush()) return code;
+    }
+    return flush();
+}
+
 int mg_linear_f16x2_pack_weight_padded(const float* W, long w_stride_o, long w_stride_i, int dim_in, int dim_out, int dim_pad,
                                        void* packed, mg_stream_t stream) {
-    MG_REQUIRE(dim_in >= 0 && dim_out >= 0 && dim_pad >= dim_in, "mg_linear_f16x2_pack_weight: bad size");
-    if (dim_in == 0 || dim_out == 0) return MG_OK;
-    MG_REQUIRE(W && packed && aligned16(packed), "mg_linear_f16x2_pack_weight: null or unaligned pointer");
-    MG_REQUIRE(dim_pad % 32 == 0, "mg_linear_f16x2_pack_weight: dim_in must be a multiple of 32");
-    const int O_pad = o_pad_of(dim_out);
-    _Float16* planes = static_cast<_Float16*>(packed);
-    float* inv = reinterpret_cast<float*>(planes + 2L * O_pad * dim_pad);
-    hipLaunchKernelGGL(pack_weight_f16x2_kernel, dim3((unsigned)(O_pad / 32)), dim3(kPackThreads), 0, (hipStream_t)stream,
-                       W, w_stride_o, w_stride_i, dim_in, dim_pad, dim_out, O_pad, planes, inv);
-    return check_launch("mg_linear_f16x2_pack_weight");
+    const mg_f16x2_weight w{W, w_stride_o, w_stride_i, dim_in, dim_out, dim_pad, packed};
+    return mg_linear_f16x2_pack_weights(&w, 1, stream);
 }
 
 int mg_linear_f16x2_pack_weight(const float* W, long w_stride_o, long w_stride_i, int dim_in, int dim_out,

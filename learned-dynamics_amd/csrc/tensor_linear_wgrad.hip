@@ -309,7 +309,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
                                                           const float* __restrict__ dy_parts, int n_dy_parts,
                                                           const float* __restrict__ x_parts, int n_x_parts,
                                                           long R, int I, int O, long rows_per_block,
-                                                          float* __restrict__ part, float* __restrict__ colsum_part) {
+                                                          float* __restrict__ part, float* __restrict__ colsum_part,
+                                                          long bias_rows) {
     // [stage buffer][operand: dy, x][piece: hi, lo][LDS row][64 bytes]
     __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kFBuf];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -346,9 +347,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         const int first_live = (int)(r - first_row(r)) - 8 * octet;                // rows u >= first_live count
         halfx8 hi[4], lo[4];
         if (sum_cols) {
+            const long last_live = bias_rows - first_row(r) - 8 * octet;           // rows u < last_live have a bias
 #pragma unroll
             for (int u = 0; u < 8; u++) {
-                const float w = (u >= first_live && r < r_hi) ? 1.f : 0.f;
+                const float w = (u >= first_live && u < last_live && r < r_hi) ? 1.f : 0.f;
                 colsum.x += w * v[u].x; colsum.y += w * v[u].y; colsum.z += w * v[u].z; colsum.w += w * v[u].w;
             }
         }
@@ -589,9 +591,9 @@ int mg_tensor_linear_wgrad_f16x2_supported(long rows, int dim_in, int dim_out) {
     return rows >= 4096 && dim_in >= 4 && dim_out >= 4 && dim_in % 4 == 0 && dim_out % 4 == 0;
 }
 
-int mg_tensor_linear_wgrad_f16x2(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,
-                                 const float* x_bound, long n_x_bound, long rows, int dim_in, int dim_out,
-                                 void* workspace, float* dW, float* db, mg_stream_t stream) {
+int mg_tensor_linear_wgrad_f16x2_rows(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,
+                                      const float* x_bound, long n_x_bound, long rows, long bias_rows, int dim_in, int dim_out,
+                                      void* workspace, float* dW, float* db, mg_stream_t stream) {
     MG_REQUIRE(mg_tensor_linear_wgrad_f16x2_supported(rows, dim_in, dim_out),
                "mg_tensor_linear_wgrad_f16x2: needs rows >= 4096 and dims that are multiples of 4");
     MG_REQUIRE(dy && x && workspace && dW, "mg_tensor_linear_wgrad_f16x2: null pointer");
@@ -627,12 +629,19 @@ int mg_tensor_linear_wgrad_f16x2(const float* dy, const float* x, const float* d
     const float* x_parts = (x_bound && n_x_bound <= kDirectBounds) ? x_bound : maxima + kFParts;
     dim3 grid((unsigned)ceil_div(dim_out, kFTile), (unsigned)ceil_div(dim_in, kFTile), (unsigned)splits), block(256);
     hipLaunchKernelGGL(wgrad_f16x2_kernel, grid, block, 0, st, dy, x, dy_parts, na, x_parts, nb, rows, dim_in, dim_out,
-                       rpb, part, colsum_part);
+                       rpb, part, colsum_part, bias_rows);
     const long n_sum = n + (db ? dim_out : 0);
     const unsigned nblocks = (unsigned)(ceil_div(n_sum, 256) < 1024 ? ceil_div(n_sum, 256) : 1024);
     hipLaunchKernelGGL(wgrad_reduce2_kernel, dim3(nblocks), dim3(256), 0, st, (const float*)part, n, dW,
                        (const float*)colsum_part, (long)(db ? dim_out : 0), db, (int)splits);
     return check_launch("mg_tensor_linear_wgrad_f16x2");
+}
+
+int mg_tensor_linear_wgrad_f16x2(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,
+                                 const float* x_bound, long n_x_bound, long rows, int dim_in, int dim_out,
+                                 void* workspace, float* dW, float* db, mg_stream_t stream) {
+    return mg_tensor_linear_wgrad_f16x2_rows(dy, x, dy_bound, n_dy_bound, x_bound, n_x_bound, rows, rows, dim_in, dim_out,
+                                             workspace, dW, db, stream);
 }
 
 int mg_tensor_linear_wgrad(int inds, const float* dy, const float* x, long rows, int dim_in, int dim_out,

@@ -34,6 +34,17 @@ public:
         Value value;
     };
 
+    // whether an entry for the current version is there (always true for tensors nothing is kept for)
+    bool has(const at::Tensor& W, int kind, int64_t extra) {
+        const at::Tensor owner = W.is_view() ? at::Tensor(W._base()) : W;
+        if (owner.is_inference()) return true;
+        c10::TensorImpl* impl = owner.unsafeGetTensorImpl();
+        std::lock_guard<std::mutex> lock(mutex_);
+        auto it = slots_.find(Key{impl, kind, extra, W.storage_offset(), W.size(0), W.size(-1), W.stride(0), W.stride(-1)});
+        return it != slots_.end() && it->second.version == impl->version_counter().current_version() &&
+               it->second.data == owner.data_ptr() && it->second.epoch == g_epoch.load();
+    }
+
     template <typename Make>
     Value get(const at::Tensor& W, int kind, int64_t extra, Make&& make) {
         const at::Tensor owner = W.is_view() ? at::Tensor(W._base()) : W;
@@ -607,6 +618,377 @@ std::tuple<at::Tensor, at::Tensor> painn_message_edges(const at::Tensor& row_ptr
     return {out_a, out_v};
 }
 
+// ------------------------------------------------------------------ PaiNN layers under differentiation
+// A value and its forward-mode tangent travel as one array of 2 R rows (values first): one launch per linear map, weight
+// gradient and activation for both.  The halves are handed out as two tensors on one storage, and taken back as one array
+// where they still lie one behind the other.
+at::Tensor on_storage(const at::Tensor& of, int64_t offset, at::IntArrayRef shape) {
+    std::vector<int64_t> strides(shape.size());
+    int64_t step = 1;
+    for (size_t k = shape.size(); k-- > 0;) {
+        strides[k] = step;
+        step *= shape[k];
+    }
+    // (not a view: the halves are written once, before they are handed out, and have version counters of their own)
+    return at::empty({0}, of.options().requires_grad(false)).set_(of.storage(), of.storage_offset() + offset, shape, strides);
+}
+OptTensor second_half(const at::Tensor& y, at::IntArrayRef shape, bool dual) {
+    return dual ? OptTensor(on_storage(y, y.numel() / 2, shape)) : OptTensor();
+}
+at::Tensor stacked(const at::Tensor& p, const OptTensor& t, int64_t cols) {
+    check_input(p, "x");
+    const int64_t rows = cols ? p.numel() / cols : 0;
+    if (!t.has_value()) return p.reshape({rows, cols});
+    check_input(*t, "tangent of x");
+    TORCH_CHECK(t->numel() == p.numel(), "a tangent must have the shape of its value");
+    if (t->storage().data() == p.storage().data() && t->storage_offset() == p.storage_offset() + p.numel())
+        return on_storage(p, 0, {2 * rows, cols});
+    return at::cat({p.reshape({rows, cols}), t->reshape({rows, cols})});
+}
+
+// packed planes of several weights that the next kernels read, those that are missing in one launch
+void pack_ahead(const Tensors& weights) {
+    if (mg_get_linear_mode() != kModeF16x2) return;
+    Tensors missing;
+    for (const at::Tensor& W : weights)
+        if (W.size(1) % 32 == 0 && W.size(1) >= 64 && W.size(0) >= 8 && !cache<at::Tensor>().has(W, 2, W.size(1))) missing.push_back(W);
+    if (missing.size() < 2) return;
+    std::vector<mg_f16x2_weight> jobs;
+    Tensors planes;
+    for (const at::Tensor& W : missing) {
+        size_t bytes = 0;
+        check(mg_linear_f16x2_packed_weight_bytes((int)W.size(1), (int)W.size(0), &bytes));
+        planes.push_back(bytes_like(W, bytes));
+        jobs.push_back({fp(W), (long)W.stride(0), (long)W.stride(1), (int)W.size(1), (int)W.size(0), (int)W.size(1),
+                        planes.back().data_ptr()});
+    }
+    check(mg_linear_f16x2_pack_weights(jobs.data(), (int)jobs.size(), stream_of(missing[0])));
+    for (size_t k = 0; k < missing.size(); k++) {
+        const at::Tensor p = planes[k];
+        cache<at::Tensor>().get(missing[k], 2, missing[k].size(1), [&] { return p; });
+    }
+}
+
+// y = x W^T, with the bias added to the first bias_rows rows; ymax: row bounds of y where the kernel that runs emits them
+at::Tensor rows_linear(const at::Tensor& W, const OptTensor& bias, const at::Tensor& x, int64_t bias_rows, Bound bound,
+                       OptTensor* ymax = nullptr) {
+    const int64_t rows = x.size(0), dim_in = W.size(1), dim_out = W.size(0);
+    at::Tensor y = floats(x, {rows, dim_out});
+    if (rows == 0) return y;
+    if (mg_get_linear_mode() == kModeF16x2 && f16x2_takes(rows, dim_in, dim_out, x)) {
+        if (!bound.base.has_value()) bound = Bound{row_absmax(x)};
+        at::Tensor m;
+        if (ymax) m = floats(x, {rows, rowmax_parts(rows, dim_in, dim_out, false)});
+        run_f16x2(W, dim_in, fp(x), rows, bound, bias, kActNone, false, 1, y, ymax ? &m : nullptr, false, bias_rows);
+        if (ymax) *ymax = m;
+        return y;
+    }
+    auto piece = [&](int64_t lo, int64_t hi, const OptTensor& b) {
+        if (hi > lo)
+            linear_fwd(0, W, x.narrow(0, lo, hi - lo), b, kActNone, OptTensor(y.narrow(0, lo, hi - lo)), false, 0, 0, OptTensor(), 1,
+                       0, 1, false, OptTensor(), OptTensor(), false);
+    };
+    const int64_t cut = bias.has_value() ? std::min(bias_rows, rows) : rows;
+    piece(0, cut, bias);
+    piece(cut, rows, OptTensor());
+    return y;
+}
+
+// dW over all rows and db over the first bias_rows
+std::pair<at::Tensor, OptTensor> rows_wgrad(const at::Tensor& dy, const at::Tensor& x, int64_t bias_rows, bool want_bias,
+                                            const OptTensor& dy_bound, const OptTensor& x_bound) {
+    const int64_t rows = x.size(0), dim_in = x.size(1), dim_out = dy.size(1);
+    if (mg_get_linear_mode() == kModeF16x2 && aligned16(x) && aligned16(dy) &&
+        mg_tensor_linear_wgrad_f16x2_supported(rows, (int)dim_in, (int)dim_out)) {
+        at::Tensor dW = floats(x, {dim_out, dim_in}), db;
+        if (want_bias) db = floats(x, {dim_out});
+        size_t n = 0;
+        check(mg_tensor_linear_wgrad_workspace_bytes(rows, (int)dim_in, (int)dim_out, &n));
+        at::Tensor ws = bytes_like(x, n);
+        check(mg_tensor_linear_wgrad_f16x2_rows(fp(dy), fp(x), fp(dy_bound), dy_bound.has_value() ? dy_bound->numel() : 0, fp(x_bound),
+                                                x_bound.has_value() ? x_bound->numel() : 0, rows, bias_rows, (int)dim_in, (int)dim_out,
+                                                ws.data_ptr(), fp(dW), want_bias ? fp(db) : nullptr, stream_of(x)));
+        return {dW, want_bias ? OptTensor(db) : OptTensor()};
+    }
+    at::Tensor dW = std::get<0>(linear_wgrad(0, dy, x, dy_bound, x_bound, false));
+    return {dW, want_bias ? OptTensor(dy.narrow(0, 0, bias_rows).sum(0)) : OptTensor()};
+}
+
+// |SiLU(z)| <= |z| and |SiLU'(z)| <= 1.0999
+constexpr float kSiluSlope = 1.1f;
+
+// Linear, SiLU, Linear, SiLU, Linear on S = [x; x_t] (R or 2 R rows): y and what the adjoint reads again
+std::pair<at::Tensor, std::vector<OptTensor>> mlp_rows_fwd(const at::Tensor& S, int64_t R, OptTensor bound, const Tensors& W,
+                                                           const Tensors& b, bool train) {
+    check_chain(S, W, b, kSiluMlp);
+    const bool dual = S.size(0) != R;
+    if (train) pack_ahead({W[0], W[1], W[2], W[0].t(), W[1].t(), W[2].t()});
+    if (!bound.has_value() && S.size(1) >= 64) bound = row_absmax(S);
+    std::vector<OptTensor> saved{bound};
+    at::Tensor h = S;
+    Bound hb{bound};
+    for (int l = 0; l < 2; l++) {
+        OptTensor m;
+        at::Tensor z = rows_linear(W[l], OptTensor(b[l]), h, R, hb, &m);
+        h = floats(z, z.sizes());
+        check(mg_silu_rows_fwd(fp(z), R, (int)z.size(1), dual, fp(h), stream_of(z)));
+        hb = Bound{m, dual ? kSiluSlope : 1.f};
+        saved.insert(saved.end(), {OptTensor(z), m, OptTensor(h)});
+    }
+    return {rows_linear(W[2], OptTensor(b[2]), h, R, hb), saved};
+}
+
+// gradients of the rows S (if wanted), then of the three weights and biases
+std::tuple<OptTensor, Tensors> mlp_rows_bwd(at::Tensor g, OptTensor g_bound, const at::Tensor& S, int64_t R, const Tensors& W,
+                                            const std::vector<OptTensor>& saved, bool want_x, bool want_params) {
+    const bool dual = S.size(0) != R;
+    Tensors params(6);
+    OptTensor g_x;
+    for (int l = 2; l >= 0; l--) {
+        if (!g_bound.has_value()) g_bound = row_absmax(g);
+        const at::Tensor& in = l == 0 ? S : *saved[3 * l];
+        const OptTensor& in_bound = l == 0 ? saved[0] : saved[3 * l - 1];
+        if (want_params) {
+            auto [dW, db] = rows_wgrad(g, in, R, true, g_bound, in_bound);
+            params[2 * l] = dW;
+            params[2 * l + 1] = *db;
+        }
+        if (l == 0) {
+            if (want_x) g_x = rows_linear(W[0].t(), OptTensor(), g, 0, Bound{g_bound});
+            break;
+        }
+        const at::Tensor dh = rows_linear(W[l].t(), OptTensor(), g, 0, Bound{g_bound});
+        const at::Tensor& z = *saved[3 * l - 2];
+        g = floats(z, z.sizes());
+        at::Tensor m = floats(z, {z.size(0), 1});
+        check(mg_silu_rows_bwd(fp(z), fp(dh), R, (int)z.size(1), dual, fp(g), fp(m), stream_of(z)));
+        g_bound = m;
+    }
+    return {g_x, params};
+}
+
+std::vector<int64_t> with_last(const at::Tensor& x, int64_t last) {
+    std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = last;
+    return shape;
+}
+
+std::tuple<at::Tensor, OptTensor, std::vector<OptTensor>> mlp_silu_fwd(const at::Tensor& x, const OptTensor& x_t, const OptTensor& bound,
+                                                                       const Tensors& W, const Tensors& b, bool train) {
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    const at::Tensor S = stacked(x, x_t, x.size(-1));
+    auto [y, saved] = mlp_rows_fwd(S, x.numel() / x.size(-1), bound, W, b, train);
+    const auto shape = with_last(x, y.size(1));
+    return {on_storage(y, 0, shape), second_half(y, shape, x_t.has_value()), saved};
+}
+
+std::tuple<OptTensor, OptTensor, Tensors> mlp_silu_bwd(const at::Tensor& g, const OptTensor& g_t, const at::Tensor& x, const OptTensor& x_t,
+                                                       const Tensors& W, const std::vector<OptTensor>& saved, bool want_x,
+                                                       bool want_params) {
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    const bool dual = x_t.has_value();
+    const at::Tensor S = stacked(x, x_t, x.size(-1)), G = stacked(g, g_t, g.size(-1));
+    auto [g_x, params] = mlp_rows_bwd(G, OptTensor(), S, x.numel() / x.size(-1), W, saved, want_x, want_params);
+    if (!want_x) return {OptTensor(), OptTensor(), params};
+    return {on_storage(*g_x, 0, x.sizes()), second_half(*g_x, x.sizes(), dual), params};
+}
+
+// enc, enc_t, row bounds of both, dir, dir_t
+std::tuple<at::Tensor, OptTensor, at::Tensor, at::Tensor, OptTensor> edge_encode_fwd(const at::Tensor& r, const OptTensor& r_t, int64_t n,
+                                                                                     double rmax, double eps) {
+    check_input(r, "r_ij");
+    TORCH_CHECK(r.dim() == 2 && r.size(1) == 3, "r_ij must have shape (edges, 3)");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(r.device());
+    const int64_t E = r.size(0), copies = r_t.has_value() ? 2 : 1;
+    if (r_t.has_value()) check_input(*r_t, "tangent of r_ij");
+    at::Tensor enc = floats(r, {copies * E, n}), bound = floats(r, {copies * E, 1}), dir = floats(r, {copies * E, 3});
+    check(mg_painn_edge_encode_fwd(fp(r), fp(r_t), E, (int)n, (float)rmax, (float)eps, fp(enc), fp(bound), fp(dir),
+                                   r_t.has_value() ? fp(dir) + 3 * E : nullptr, stream_of(r)));
+    const bool dual = r_t.has_value();
+    return {on_storage(enc, 0, {E, n}), second_half(enc, {E, n}, dual), bound, on_storage(dir, 0, {E, 3}), second_half(dir, {E, 3}, dual)};
+}
+
+std::tuple<at::Tensor, OptTensor> edge_encode_bwd(const at::Tensor& r, const OptTensor& r_t, int64_t n, double rmax, double eps,
+                                                  const at::Tensor& g_enc, const OptTensor& g_enc_t, const at::Tensor& g_dir,
+                                                  const OptTensor& g_dir_t) {
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(r.device());
+    const bool dual = r_t.has_value();
+    const at::Tensor G = stacked(g_enc, g_enc_t, n);
+    check_input(g_dir, "g_dir");
+    if (dual) check_input(*g_dir_t, "g_dir_t");
+    at::Tensor g_r = floats(r, r.sizes()), g_rt;
+    if (dual) g_rt = floats(r, r.sizes());
+    check(mg_painn_edge_encode_bwd(fp(r), fp(r_t), r.size(0), (int)n, (float)rmax, (float)eps, fp(G), fp(g_dir), fp(g_dir_t), fp(g_r),
+                                   dual ? fp(g_rt) : nullptr, stream_of(r)));
+    return {g_r, dual ? OptTensor(g_rt) : OptTensor()};
+}
+
+// in: dist, dist_t, actv, actv_t, v, v_t, dir, dir_t (the odd ones may be missing)
+mg_painn_combine_dual combine_in(const std::vector<OptTensor>& in) {
+    TORCH_CHECK(in.size() == 8, "combine_dual: eight operands expected");
+    for (int k = 0; k < 8; k++) {
+        TORCH_CHECK(k % 2 == 1 || in[k].has_value(), "combine_dual: a value is missing");
+        if (in[k].has_value()) check_input(*in[k], "operand of the message");
+        TORCH_CHECK(k % 2 == 0 || !in[k].has_value() || in[k]->numel() == in[k - 1]->numel(), "a tangent must have the shape of its value");
+    }
+    const int64_t E = in[6]->size(0), rows = in[4]->size(0), n = in[4]->size(1);
+    TORCH_CHECK(in[0]->dim() == 2 && in[0]->size(0) == E && in[0]->size(1) == 4 * n && in[6]->size(1) == 3 && in[2]->dim() == 2 &&
+                    in[2]->size(0) == rows && in[2]->size(1) == 4 * n && in[4]->dim() == 3 && in[4]->size(2) == 3,
+                "combine_dual: dist (edges, 4n), actv (nodes, 4n), v (nodes, n, 3) and dir (edges, 3) expected");
+    return {fp(in[0]), fp(in[1]), fp(in[2]), fp(in[3]), fp(in[4]), fp(in[5]), fp(in[6]), fp(in[7]), E, rows, (int)n};
+}
+
+Tensors combine_dual_fwd(const std::vector<OptTensor>& in, const at::Tensor& node, const at::Tensor& row_ptr, int64_t n_out) {
+    const mg_painn_combine_dual a = combine_in(in);
+    check_input(node, "node", at::kInt);
+    check_input(row_ptr, "row_ptr", at::kInt);
+    TORCH_CHECK(node.numel() == a.E && row_ptr.numel() == n_out + 1, "combine_dual: index sizes");
+    const at::Tensor& like = *in[0];
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(like.device());
+    at::Tensor v = floats(like, {2 * n_out, a.n, 3}), s = floats(like, {2 * n_out, a.n});
+    check(mg_painn_combine_dual_fwd(&a, node.data_ptr<int>(), row_ptr.data_ptr<int>(), n_out, fp(v), fp(v) + n_out * a.n * 3, fp(s),
+                                    fp(s) + n_out * a.n, stream_of(like)));
+    const std::vector<int64_t> sv{n_out, a.n, 3}, sa{n_out, a.n};
+    return {on_storage(v, 0, sv), on_storage(s, 0, sa), *second_half(v, sv, true), *second_half(s, sa, true)};
+}
+
+std::vector<OptTensor> combine_dual_bwd(const std::vector<OptTensor>& in, const at::Tensor& row_ptr, const OptTensor& order,
+                                        const Tensors& g, const at::Tensor& grad_row, int64_t n_grad_rows, const std::vector<bool>& want) {
+    const mg_painn_combine_dual a = combine_in(in);
+    check_input(row_ptr, "row_ptr", at::kInt);
+    check_input(grad_row, "grad_row", at::kInt);
+    if (order.has_value()) check_input(*order, "order", at::kInt);
+    TORCH_CHECK(row_ptr.numel() == a.n_rows + 1 && grad_row.numel() == a.E && (!order.has_value() || order->numel() == a.E) &&
+                    g.size() == 4 && want.size() == 8,
+                "combine_dual: index sizes");
+    for (int k = 0; k < 4; k++) {
+        check_input(g[k], "gradient of the message");
+        TORCH_CHECK(g[k].numel() == n_grad_rows * a.n * (k % 2 == 0 ? 3 : 1), "combine_dual: gradient sizes");
+    }
+    const at::Tensor& like = *in[0];
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(like.device());
+    std::vector<OptTensor> out(8);
+    float* p[8];
+    for (int k = 0; k < 8; k += 2) {             // a value's gradient and its tangent's, one behind the other
+        p[k] = p[k + 1] = nullptr;
+        const auto shape = in[k]->sizes();
+        const bool first = want[k] || (k == 6 && want[7]), second = want[k + 1] && in[k + 1].has_value();
+        if (!first && !second) continue;
+        std::vector<int64_t> both(shape.begin(), shape.end());
+        both[0] *= 2;
+        at::Tensor buf = floats(like, both);
+        if (first) out[k] = on_storage(buf, 0, shape);
+        if (second) out[k + 1] = on_storage(buf, in[k]->numel(), shape);
+        p[k] = first ? fp(buf) : nullptr;
+        p[k + 1] = second ? fp(buf) + in[k]->numel() : nullptr;
+    }
+    const mg_painn_combine_dual_grad d{p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7]};
+    check(mg_painn_combine_dual_bwd(&a, row_ptr.data_ptr<int>(), order.has_value() ? order->data_ptr<int>() : nullptr, fp(g[0]),
+                                    fp(g[2]), fp(g[1]), fp(g[3]), grad_row.data_ptr<int>(), n_grad_rows, &d, stream_of(like)));
+    return out;
+}
+
+// x_v (and its tangent) as one plain row per (row, component), and the row maxima
+std::pair<at::Tensor, at::Tensor> vector_rows(const at::Tensor& x_v, const OptTensor& x_vt, int64_t R, int64_t n) {
+    const int64_t copies = x_vt.has_value() ? 2 : 1;
+    if (n >= 32 && n <= 256 && power_of_two(n)) {
+        at::Tensor x2 = floats(x_v, {copies * R * 3, n}), m = floats(x_v, {copies * R * 3, 1});
+        check(mg_components_to_rows(fp(x_v), R, (int)n, 3, (int)n, fp(x2), fp(m), stream_of(x_v)));
+        if (x_vt.has_value())
+            check(mg_components_to_rows(fp(*x_vt), R, (int)n, 3, (int)n, fp(x2) + R * 3 * n, fp(m) + R * 3, stream_of(x_v)));
+        return {x2, m};
+    }
+    at::Tensor x2 = stacked(x_v, x_vt, n * 3).reshape({copies * R, n, 3}).transpose(1, 2).contiguous().reshape({copies * R * 3, n});
+    return {x2, row_absmax(x2)};
+}
+
+// Update.forward with its adjoint's operands: x_a (batch, nodes, n), x_v (batch, nodes, n, 3), weights {l, r, v}
+std::tuple<Tensors, std::vector<OptTensor>> painn_update_train_fwd(const at::Tensor& x_a, const OptTensor& x_at, const at::Tensor& x_v,
+                                                                   const OptTensor& x_vt, const Tensors& lrv_W, const Tensors& W,
+                                                                   const Tensors& b, int groups, const at::Tensor& gamma,
+                                                                   const at::Tensor& beta, double eps) {
+    check_input(x_a, "x_a");
+    check_input(x_v, "x_v");
+    check_input(gamma, "gamma");
+    check_input(beta, "beta");
+    const int64_t B = x_a.size(0), N = x_a.size(1), n = x_a.size(2), R = B * N;
+    TORCH_CHECK(x_v.numel() == 3 * x_a.numel() && gamma.numel() == n && beta.numel() == n, "painn_update: operand sizes");
+    const bool dual = x_vt.has_value();
+    for (const OptTensor& t : {x_at, x_vt})
+        if (t.has_value()) check_input(*t, "tangent");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x_a.device());
+    const int64_t copies = dual ? 2 : 1;
+    const at::Tensor W_lrv = at::cat(lrv_W);
+    pack_ahead({W_lrv, W_lrv.t(), W[0], W[1], W[2], W[0].t(), W[1].t(), W[2].t()});
+    auto [x2, x2max] = vector_rows(x_v, x_vt, R, n);
+    const at::Tensor lrv = rows_linear(W_lrv, OptTensor(), x2, 0, Bound{OptTensor(x2max)});
+    at::Tensor ip = floats(x_a, {copies * R, n}), cat = floats(x_a, {copies * R, 2 * n}), cat_max = floats(x_a, {copies * R, 1});
+    const mg_stream_t st = stream_of(x_a);
+    check(mg_painn_update_pre_fwd(fp(lrv), fp(x_a), fp(x_at), R, (int)n, dual, fp(ip), fp(cat), fp(cat_max), st));
+    auto [y, mlp_saved] = mlp_rows_fwd(cat, R, OptTensor(cat_max), W, b, false);
+    TORCH_CHECK(y.size(1) == 3 * n, "the update's MLP must end in 3n columns");
+    long fwd = 0, bwd = 0;
+    check(mg_painn_update_scratch_floats((int)B, (int)N, (int)n, groups, &fwd, &bwd));
+    at::Tensor scratch = floats(x_a, {std::max<int64_t>(fwd, 1)}), stats = floats(x_a, {B * groups, 4});
+    at::Tensor out_a = floats(x_a, {copies * R, n}), out_v = floats(x_a, {copies * R, n, 3});
+    check(mg_painn_update_post_fwd(fp(lrv), fp(ip), fp(y), fp(gamma), fp(beta), (int)B, (int)N, (int)n, groups, (float)eps, dual,
+                                   fp(scratch), fp(stats), fp(out_a), fp(out_v), st));
+    Tensors out{on_storage(out_a, 0, x_a.sizes()), on_storage(out_v, 0, x_v.sizes())};
+    if (dual) {
+        out.push_back(*second_half(out_a, x_a.sizes(), true));
+        out.push_back(*second_half(out_v, x_v.sizes(), true));
+    }
+    std::vector<OptTensor> saved{OptTensor(W_lrv), OptTensor(x2), OptTensor(x2max), OptTensor(lrv), OptTensor(ip), OptTensor(cat),
+                                 OptTensor(y), OptTensor(stats)};
+    saved.insert(saved.end(), mlp_saved.begin(), mlp_saved.end());
+    return {out, saved};
+}
+
+// gradients of x_a, x_v and their tangents, of l, r, v, of gamma and beta, and of the MLP's weights and biases
+std::tuple<std::vector<OptTensor>, Tensors> painn_update_train_bwd(const at::Tensor& g_a, const OptTensor& g_at, const at::Tensor& g_v,
+                                                                   const OptTensor& g_vt, const Tensors& W, int groups,
+                                                                   const at::Tensor& gamma, const std::vector<OptTensor>& saved) {
+    const bool dual = g_at.has_value();
+    check_input(g_a, "gradient of out_a");
+    check_input(g_v, "gradient of out_v");
+    for (const OptTensor& t : {g_at, g_vt})
+        if (t.has_value()) check_input(*t, "gradient of a tangent");
+    const int64_t B = g_a.size(0), N = g_a.size(1), n = g_a.size(2), R = B * N, copies = dual ? 2 : 1;
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(g_a.device());
+    const at::Tensor &W_lrv = *saved[0], &x2 = *saved[1], &lrv = *saved[3], &ip = *saved[4], &cat = *saved[5], &y = *saved[6],
+                     &stats = *saved[7];
+    const std::vector<OptTensor> mlp_saved(saved.begin() + 8, saved.end());
+    const mg_stream_t st = stream_of(g_a);
+    long fwd = 0, bwd = 0;
+    check(mg_painn_update_scratch_floats((int)B, (int)N, (int)n, groups, &fwd, &bwd));
+    at::Tensor scratch = floats(g_a, {std::max<int64_t>(bwd, 1)});
+    at::Tensor g_y = floats(y, y.sizes()), g_y_max = floats(y, {y.size(0), 1}), g_ip = floats(ip, ip.sizes());
+    at::Tensor g_lrv = floats(lrv, lrv.sizes()), g_lrv_max = floats(lrv, {copies * R * 3, 1});
+    at::Tensor d_gamma = floats(g_a, {n}), d_beta = floats(g_a, {n});
+    check(mg_painn_update_post_bwd(fp(lrv), fp(ip), fp(y), fp(stats), fp(gamma), fp(g_a), fp(g_at), fp(g_v), fp(g_vt), (int)B, (int)N,
+                                   (int)n, groups, dual, fp(scratch), fp(g_y), fp(g_y_max), fp(g_ip), fp(g_lrv), fp(d_gamma),
+                                   fp(d_beta), st));
+    auto [g_cat, mlp_params] = mlp_rows_bwd(g_y, OptTensor(g_y_max), cat, R, W, mlp_saved, true, true);
+    at::Tensor g_xa = floats(g_a, {copies * R, n});
+    check(mg_painn_update_pre_bwd(fp(lrv), fp(g_ip), fp(*g_cat), R, (int)n, dual, fp(g_lrv), fp(g_lrv_max), fp(g_xa), st));
+    const OptTensor g_bound(g_lrv_max);
+    const at::Tensor dW = rows_wgrad(g_lrv, x2, 0, false, g_bound, saved[2]).first;
+    at::Tensor g_xv;
+    const at::Tensor back = W_lrv.t();
+    if (mg_get_linear_mode() == kModeF16x2 && f16x2_takes(copies * R * 3, 3 * n, n, g_lrv)) {
+        g_xv = floats(g_a, {copies * R, n, 3});
+        run_f16x2(back, 3 * n, fp(g_lrv), copies * R * 3, Bound{g_bound}, OptTensor(), kActNone, false, 3, g_xv, nullptr, false);
+    } else {
+        g_xv = rows_linear(back, OptTensor(), g_lrv, 0, Bound{g_bound}).reshape({copies * R, 3, n}).transpose(1, 2).contiguous();
+    }
+    const std::vector<int64_t> sv{B, N, n, 3};
+    std::vector<OptTensor> g_x{OptTensor(on_storage(g_xa, 0, g_a.sizes())), second_half(g_xa, g_a.sizes(), dual),
+                               OptTensor(on_storage(g_xv, 0, sv)), second_half(g_xv, sv, dual)};
+    Tensors params{on_storage(dW, 0, {n, n}), on_storage(dW, n * n, {n, n}), on_storage(dW, 2 * n * n, {n, n}), d_gamma, d_beta};
+    params.insert(params.end(), mlp_params.begin(), mlp_params.end());
+    return {g_x, params};
+}
+
 }  // namespace
 
 void register_ops(pybind11::module_& m) {
@@ -623,4 +1005,12 @@ void register_ops(pybind11::module_& m) {
     m.def("painn_update", &painn_update);
     m.def("painn_message_grid", &painn_message_grid);
     m.def("painn_message_edges", &painn_message_edges);
+    m.def("mlp_silu_fwd", &mlp_silu_fwd);
+    m.def("mlp_silu_bwd", &mlp_silu_bwd);
+    m.def("edge_encode_fwd", &edge_encode_fwd);
+    m.def("edge_encode_bwd", &edge_encode_bwd);
+    m.def("combine_dual_fwd", &combine_dual_fwd);
+    m.def("combine_dual_bwd", &combine_dual_bwd);
+    m.def("painn_update_train_fwd", &painn_update_train_fwd);
+    m.def("painn_update_train_bwd", &painn_update_train_bwd);
 }

@@ -171,13 +171,113 @@ def silu(z):
     return F.silu(z)
 
 
-def mlp_silu(mlp, x):
-    """painn.MLP: Linear, SiLU, Linear, SiLU, Linear (archs/meanflow_painn8.py:38-51).  |SiLU(z)| <= |z|: the row
-    maxima that a layer's kernel emits for z bound the next layer's input."""
+def _unpack(x):
+    """(value, forward-mode tangent or None) of a tensor."""
+    if getattr(fwAD, "_current_level", 0) < 0:
+        return x, None
+    p, t = fwAD.unpack_dual(x)
+    return p, t
+
+
+def _dual(p, t):
+    return p if t is None else fwAD.make_dual(p, t)
+
+
+def _dense(t):
+    return t if t is None else t.contiguous()
+
+
+def _as_pair(f, x, x_t):
+    """(value, tangent) of f, which maps one tensor to one tensor, from the plain tensors (x, x_t); x_t may be None."""
+    if x_t is None:
+        return (f(x),)
+    if getattr(fwAD, "_current_level", 0) >= 0:
+        return fwAD.unpack_dual(f(fwAD.make_dual(x, x_t)))
+    with fwAD.dual_level():
+        return tuple(fwAD.unpack_dual(f(fwAD.make_dual(x, x_t))))
+
+
+def _recorded_gradients(f, inputs, needed, grads):
+    """The gradients of f's outputs for `inputs`, recorded so that they can be differentiated again: what the fused
+    functions below fall back on inside a recorded backward pass.  f is the same layer out of differentiable pieces."""
+    with torch.enable_grad():
+        leaves = [t if t is None or t.requires_grad or not need else t.detach().requires_grad_()
+                  for t, need in zip(inputs, needed)]
+        pairs = [(o, g) for o, g in zip(f(*leaves), grads) if g is not None and o is not None and o.requires_grad]
+        wanted = [t for t, need in zip(leaves, needed) if need]
+        found = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs], create_graph=True,
+                                         allow_unused=True) if wanted and pairs else [None] * len(wanted))
+    return tuple(next(found) if need else None for need in needed)
+
+
+class _MlpSilu(torch.autograd.Function):
+    """painn.MLP on rows, values alone or values and tangents: one call into the C++ binding for each direction (three
+    linear maps and two activations; three weight gradients, two or three input gradients, two activations).  The
+    value and its tangent are two arguments and two results: forward mode is spelled out here, not left to jvp rules.
+    bound: row maxima of |x| (and of the tangent's rows) if the caller holds them."""
+
+    @staticmethod
+    def forward(ctx, x, x_t, bound, *params):
+        ctx.save_for_backward(x, x_t, *params)
+        train = any(ctx.needs_input_grad)
+        y, y_t, saved = ops.mlp_silu_fwd(x, x_t, bound, params[0::2], params[1::2], train)
+        ctx.rows_saved = saved if train else None
+        ctx.set_materialize_grads(False)
+        return y if x_t is None else (y, y_t)
+
+    @staticmethod
+    def backward(ctx, g, g_t=None):
+        x, x_t, *params = ctx.saved_tensors
+        need = list(ctx.needs_input_grad)
+        if g is None and g_t is None:
+            return (None,) * len(need)
+        if torch.is_grad_enabled():
+            outs = _recorded_gradients(lambda x, x_t, *p: _as_pair(lambda z: _mlp_rows(p, z), x, x_t), (x, x_t, *params),
+                                       need[:2] + need[3:], (g, g_t))
+            return outs[:2] + (None,) + outs[2:]
+        # (a result that nothing depends on leaves what only it depends on without a gradient, as separate functions would)
+        if g is None:
+            g, need[8] = torch.zeros_like(g_t), False                       # the last bias
+        if x_t is not None and g_t is None:
+            g_t, need[1] = torch.zeros_like(g), False
+        g_x, g_xt, d_params = ops.mlp_silu_bwd(g.contiguous(), _dense(g_t), x, x_t, params[0::2], ctx.rows_saved,
+                                               need[0] or need[1], any(need[3:]))
+        return (g_x if need[0] else None, g_xt if need[1] else None, None) \
+            + tuple(d if nd else None for d, nd in zip(d_params, need[3:]))
+
+
+def _mlp_rows(params, x):
+    """Linear, SiLU, Linear, SiLU, Linear out of differentiable pieces.  |SiLU(z)| <= |z|: the row maxima that a layer's
+    kernel emits for z bound the next layer's input."""
+    W0, b0, W1, b1, W2, b2 = params
+    lead, x = x.shape[:-1], x.reshape(-1, x.shape[-1])
+    z, b = tensor_linear(0, W0, x, bias=b0, want_bound=True)
+    z, b = tensor_linear(0, W1, silu(z), bias=b1, x_bound=b, want_bound=True)
+    return tensor_linear(0, W2, silu(z), bias=b2, x_bound=b).reshape(*lead, -1)
+
+
+def _mlp_parameters(mlp):
     L = mlp.layers
-    z, b = linear(L[0], x, want_bound=True, sequential=False)
-    z, b = linear(L[2], silu(z), x_bound=b, want_bound=True, sequential=False)
-    return linear(L[4], silu(z), x_bound=b, sequential=False)
+    return [p for k in (0, 2, 4) for p in (L[k].weight, L[k].bias)]
+
+
+def _fused(params, *tensors):
+    """Whether the fused functions take these: float32 on the device, rows of whole 16-byte pieces, no tangents on the
+    parameters."""
+    return (all(t is None or (t.is_cuda and t.dtype == torch.float32 and t.data_ptr() % 16 == 0 and t.numel() > 0) for t in tensors)
+            and all(p.is_cuda and p.dtype == torch.float32 and p.is_contiguous() and p.shape[0] % 4 == 0 for p in params)
+            and not any(has_tangent(p) for p in params))
+
+
+def mlp_silu(mlp, x):
+    """painn.MLP: Linear, SiLU, Linear, SiLU, Linear (archs/meanflow_painn8.py:38-51)."""
+    params = _mlp_parameters(mlp)
+    p, t = _unpack(x)
+    p, t = p.contiguous(), _dense(t)
+    if not (_fused(params, p, t) and p.shape[-1] % 4 == 0):
+        return _mlp_rows(params, x)
+    out = _MlpSilu.apply(p, t, None, *params)
+    return out if t is None else fwAD.make_dual(*out)
 
 
 def mlp_leaky(mlp, x):
@@ -230,13 +330,14 @@ def tens_sigmoid(inds, x):
     return x / torch.sqrt(add(xx, 1.0))
 
 
-def scal_group_norm(gn, x):
+def scal_group_norm(gn, x, gamma=None, beta=None):
     """managan/layers_common.py:201-223"""
+    gamma, beta = gn.gamma if gamma is None else gamma, gn.beta if beta is None else beta
     B, N, chan = x.shape
     xg = x.reshape(B, N, gn.groups, -1)
     sh = xg - xg.mean([1, 3], keepdim=True)
     var = (sh ** 2).mean([1, 3], keepdim=True)
-    return add(mul((sh / torch.sqrt(add(var, gn.epsilon))).reshape(B, N, chan), gn.gamma), gn.beta)
+    return add(mul((sh / torch.sqrt(add(var, gn.epsilon))).reshape(B, N, chan), gamma), beta)
 
 
 def tens_group_norm(gn, x):
@@ -369,6 +470,37 @@ class _PainnCombineGrad(torch.autograd.Function):
                         grads[j].append(outs[j])
         return ((out_g_v, out_g_a) + tuple(_sum_opt(g) if nd else None for g, nd in zip(grads, need[2:6]))
                 + (None, None, None, None))
+
+
+class _PainnCombineDual(torch.autograd.Function):
+    """_PainnCombine of values and tangents at once: (dist, dist_t, actv, actv_t, v, v_t, direction, direction_t) -> (out_v,
+    out_a, out_v_t, out_a_t), any tangent None.  One kernel each way, where the rule of _PainnCombine.jvp makes one call
+    for the values and one for each argument with a tangent, and as many in the backward pass."""
+
+    @staticmethod
+    def forward(ctx, by_dst, by_src, *args):
+        ctx.by_dst, ctx.by_src = by_dst, by_src
+        ctx.save_for_backward(*args)
+        return ops.painn_combine_dual_fwd(args, by_dst.index, by_src.row_ptr, by_src.n_rows)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        args, need = ctx.saved_tensors, ctx.needs_input_grad[2:]
+        by_dst, by_src = ctx.by_dst, ctx.by_src
+        if torch.is_grad_enabled():
+            return (None, None) + _recorded_gradients(lambda *a: _combine_pairs(a, by_dst, by_src), args, need, grads)
+        outs = ops.painn_combine_dual_bwd(args, by_dst.row_ptr, by_dst.perm, [g.contiguous() for g in grads], by_src.index,
+                                          by_src.n_rows, need)
+        return (None, None) + tuple(o if nd else None for o, nd in zip(outs, need))
+
+
+def _combine_pairs(args, by_dst, by_src):
+    """_PainnCombineDual out of calls of _PainnCombine."""
+    values, tangents = args[0::2], args[1::2]
+    out_v, out_a = _PainnCombine.apply(*values, by_dst, by_src, _TERMS_ALL)
+    pairs = [_PainnCombine.apply(*(t if j == k else v for j, v in enumerate(values)), by_dst, by_src, terms)
+             for k, (t, terms) in enumerate(zip(tangents, (_TERMS_ALL, _TERMS_ALL, _TERMS_V, _TERMS_DIR))) if t is not None]
+    return out_v, out_a, _sum_opt([p[0] for p in pairs]), _sum_opt([p[1] for p in pairs])
 
 
 def painn_combine(graph, dist, actv_node, v_node, direction):
@@ -511,6 +643,64 @@ def _unit_vectors(r_ij, epsilon):
     return r_ij / torch.sqrt(add((r_ij ** 2).sum(-1, keepdim=True), epsilon))
 
 
+class _EdgeEncode(torch.autograd.Function):
+    """Edge vectors -> (radial_encode, unit vectors, row bounds of the encoding) and, with tangents, (radial_encode, its
+    tangent, unit vectors, their tangent, row bounds): one kernel each way."""
+
+    @staticmethod
+    def forward(ctx, r, r_t, n, rmax, epsilon):
+        ctx.save_for_backward(r, r_t)
+        ctx.shape_args = (n, rmax, epsilon)
+        enc, enc_t, bound, direction, direction_t = ops.painn_edge_encode_fwd(r, r_t, n, rmax, epsilon)
+        ctx.mark_non_differentiable(bound)
+        return (enc, direction, bound) if r_t is None else (enc, enc_t, direction, direction_t, bound)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        r, r_t = ctx.saved_tensors
+        n, rmax, epsilon = ctx.shape_args
+        need = ctx.needs_input_grad[:2]
+        if torch.is_grad_enabled():
+            def pieces(r, r_t):
+                enc = _as_pair(lambda x: radial_encode_painn(x, n, rmax), r, r_t)
+                return enc + _as_pair(lambda x: _unit_vectors(x, epsilon), r, r_t)
+            return _recorded_gradients(pieces, (r, r_t), need, grads[:-1]) + (None, None, None)
+        g = [g.contiguous() for g in grads[:-1]]
+        g_enc, g_enc_t, g_dir, g_dir_t = (g[0], None, g[1], None) if r_t is None else g
+        g_r, g_rt = ops.painn_edge_encode_bwd(r, r_t, n, rmax, epsilon, g_enc, g_enc_t, g_dir, g_dir_t)
+        return g_r if need[0] else None, g_rt if need[1] else None, None, None, None
+
+
+def _message_edges(msg, graph, actv, x_v, r_ij):
+    """The message with the filter MLP on every edge, or None where the fused functions do not take it."""
+    params, n = _mlp_parameters(msg.mlp_dist), msg.n
+    (r, r_t), (a, a_t), (v, v_t) = _unpack(r_ij), _unpack(actv), _unpack(x_v)
+    r, r_t = r.contiguous(), _dense(r_t)
+    flat = [_dense(t if t is None else gl._flat_nodes(graph, t)) for t in (a, a_t, v, v_t)]
+    if not (ops.painn_combine_supported(n) and msg.n_rbf % 4 == 0 and _fused(params, r, r_t, *flat)):
+        return None
+    if r_t is None:
+        enc, direction, bound = _EdgeEncode.apply(r, None, msg.n_rbf, msg.r0, msg.epsilon)
+        dist, dist_t, direction_t = _MlpSilu.apply(enc, None, bound, *params), None, None
+    else:
+        enc, enc_t, direction, direction_t, bound = _EdgeEncode.apply(r, r_t, msg.n_rbf, msg.r0, msg.epsilon)
+        dist, dist_t = _MlpSilu.apply(enc, enc_t, bound, *params)
+    return _combine_flat(graph, dist, dist_t, *flat, direction, direction_t)
+
+
+def _combine_flat(graph, dist, dist_t, a, a_t, v, v_t, direction, direction_t):
+    """(out_a, out_v), with tangents where an operand has one, from operands per edge and per flat node."""
+    if all(t is None for t in (dist_t, a_t, v_t, direction_t)):
+        pairs = [(o, None) for o in _PainnCombine.apply(dist, a, v, direction, graph.by_dst, graph.by_src, _TERMS_ALL)]
+    else:
+        o_v, o_a, o_vt, o_at = _PainnCombineDual.apply(graph.by_dst, graph.by_src, dist, dist_t, a, a_t, v, v_t, direction,
+                                                       direction_t)
+        pairs = [(o_v, o_vt), (o_a, o_at)]
+    out_v, out_a = (_dual(*(t if t is None else t.reshape(graph.batch, graph.nodes, *t.shape[1:]) for t in pair))
+                    for pair in pairs)
+    return out_a, out_v
+
+
 _SLICE_PERMUTATIONS = {}
 
 
@@ -591,20 +781,88 @@ def painn_message(msg, graph, x_a, x_v, r_ij):
                                                2.0 * msg.r0, msg.epsilon)
         return (out_a.reshape(graph.batch, graph.nodes, *out_a.shape[1:]),
                 out_v.reshape(graph.batch, graph.nodes, *out_v.shape[1:]))
-    dist = painn_filter(msg, r_ij)
-    out_v, out_a = painn_combine(graph, dist, actv, x_v, _unit_vectors(r_ij, msg.epsilon))
+    if not rows and not getattr(graph, "padded", False):
+        out = _message_edges(msg, graph, actv, x_v, r_ij)
+        if out is not None:
+            return out
+    dist, direction = painn_filter(msg, r_ij), _unit_vectors(r_ij, msg.epsilon)
+    if ops.painn_combine_supported(n) and any(has_tangent(t) for t in (actv, x_v)) and not has_tangent(dist):
+        flat = [_dense(t if t is None else gl._flat_nodes(graph, t)) for t in (*_unpack(actv), *_unpack(x_v))]
+        if all(t is None or t.data_ptr() % 16 == 0 for t in (*flat, dist)):
+            return _combine_flat(graph, dist.contiguous(), None, *flat, direction.contiguous(), None)
+    out_v, out_a = painn_combine(graph, dist, actv, x_v, direction)
     return out_a, out_v
+
+
+class _PainnUpdate(torch.autograd.Function):
+    """painn.Update, values alone or values and tangents: one call into the C++ binding for each direction."""
+
+    @staticmethod
+    def forward(ctx, upd, x_a, x_at, x_v, x_vt, *params):
+        ctx.upd = upd
+        ctx.save_for_backward(x_a, x_at, x_v, x_vt, *params)
+        outs, saved = ops.painn_update_train_fwd(x_a, x_at, x_v, x_vt, params[:3], params[5::2], params[6::2], upd.gn.groups,
+                                                 params[3], params[4], upd.gn.epsilon)
+        ctx.rows_saved = saved if any(ctx.needs_input_grad) else None
+        ctx.set_materialize_grads(False)
+        return tuple(outs)
+
+    @staticmethod
+    def backward(ctx, g_a, g_v, g_at=None, g_vt=None):
+        upd, need = ctx.upd, list(ctx.needs_input_grad)
+        x_a, x_at, x_v, x_vt, *params = ctx.saved_tensors
+        if all(g is None for g in (g_a, g_v, g_at, g_vt)):
+            return (None,) * len(need)
+        if torch.is_grad_enabled():
+            def pieces(x_a, x_at, x_v, x_vt, *params):
+                if x_vt is None:
+                    return _update_pieces(upd, params, x_a, x_v)
+                split = lambda: tuple(zip(*(fwAD.unpack_dual(o) for o in _update_pieces(upd, params, _dual(x_a, x_at), _dual(x_v, x_vt)))))
+                if getattr(fwAD, "_current_level", 0) >= 0:
+                    return sum(split(), ())
+                with fwAD.dual_level():
+                    return sum(split(), ())
+            return (None,) + _recorded_gradients(pieces, (x_a, x_at, x_v, x_vt, *params), need[1:], (g_a, g_v, g_at, g_vt))
+        # (a result that nothing depends on leaves what only it depends on without a gradient, as separate functions would)
+        if g_a is None and g_at is None:
+            need[5] = need[8] = need[9] = False                             # the map l, gamma, beta
+        if g_v is None and g_vt is None:
+            need[7] = False                                                 # the map v
+        if g_a is None:
+            need[9] = False
+        zeros = lambda g, like: torch.zeros_like(like) if g is None else g.contiguous()
+        g_a, g_v = zeros(g_a, x_a), zeros(g_v, x_v)
+        if x_vt is not None:
+            g_at, g_vt = zeros(g_at, x_a), zeros(g_vt, x_v)
+        g_x, d_params = ops.painn_update_train_bwd(g_a, g_at, g_v, g_vt, params[5::2], upd.gn.groups, params[3], ctx.rows_saved)
+        grads = list(g_x) + list(d_params)
+        return (None,) + tuple(g if nd else None for g, nd in zip(grads, need[1:]))
+
+
+def _update_pieces(upd, params, x_a, x_v):
+    """painn.Update out of differentiable pieces"""
+    n = upd.n
+    W_l, W_r, W_v = params[:3]
+    x_v = x_v.contiguous()
+    v_l, v_r = (tensor_linear(1, W, x_v) for W in (W_l, W_r))
+    ip = (v_l * v_r).sum(-1)
+    y = _mlp_rows(params[5:], torch.cat([x_a, torch.linalg.vector_norm(v_r, dim=-1)], dim=-1))
+    v = tensor_linear(1, W_v, x_v) * y[..., :n, None]
+    a = scal_group_norm(upd.gn, ip * y[..., n:2 * n], params[3], params[4]) + y[..., 2 * n:]
+    return a, v / torch.sqrt(add((v ** 2).sum(-1, keepdim=True), 1.))
 
 
 def painn_update(upd, x_a, x_v):
     """archs/meanflow_painn8.py:63-75"""
-    n = upd.n
-    v_l, v_r = upd.lin_l(x_v), upd.lin_r(x_v)
-    ip = (v_l * v_r).sum(-1)
-    y = mlp_silu(upd.mlp, torch.cat([x_a, torch.linalg.vector_norm(v_r, dim=-1)], dim=-1))
-    v = upd.lin_v(x_v) * y[..., :n, None]
-    a = scal_group_norm(upd.gn, ip * y[..., n:2 * n]) + y[..., 2 * n:]
-    return a, v / torch.sqrt(add((v ** 2).sum(-1, keepdim=True), 1.))
+    params = [upd.lin_l.W, upd.lin_r.W, upd.lin_v.W, upd.gn.gamma, upd.gn.beta, *_mlp_parameters(upd.mlp)]
+    pairs = [tuple(_dense(t) for t in _unpack(x)) for x in (x_a, x_v)]
+    (a, a_t), (v, v_t) = pairs
+    if a_t is not None and v_t is None:
+        v_t = torch.zeros_like(v)
+    if not (x_a.dim() == 3 and upd.n <= 256 and _fused(params, a, a_t, v, v_t)):
+        return _update_pieces(upd, params, x_a, x_v)
+    outs = _PainnUpdate.apply(upd, a, a_t, v, v_t, *params)
+    return outs if v_t is None else tuple(fwAD.make_dual(p, t) for p, t in zip(outs[:2], outs[2:]))
 
 
 def apply_tens_prod_submodules(module, prods):

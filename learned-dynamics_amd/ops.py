@@ -1181,6 +1181,21 @@ def tensor_linear_wgrad(inds, dy, x, dy_bound=None, x_bound=None, want_bias=Fals
     return (dW, db) if want_bias else dW
 
 
+# ------------------------------------------------- PaiNN layers under differentiation (values, or values and tangents)
+mlp_silu_fwd = _ext.mlp_silu_fwd
+mlp_silu_bwd = _ext.mlp_silu_bwd
+painn_edge_encode_fwd = _ext.edge_encode_fwd
+painn_edge_encode_bwd = _ext.edge_encode_bwd
+painn_combine_dual_bwd = _ext.combine_dual_bwd
+painn_update_train_fwd = _ext.painn_update_train_fwd
+painn_update_train_bwd = _ext.painn_update_train_bwd
+
+
+def painn_combine_dual_fwd(args, node, row_ptr, n_out):
+    """(dist, dist_t, actv, actv_t, v, v_t, direction, direction_t), tangents or None -> (out_v, out_a, out_v_t, out_a_t)."""
+    return tuple(_ext.combine_dual_fwd(args, node, row_ptr, n_out))
+
+
 # ------------------------------------------------- bf16-storage configuration
 def _check_bf16(t, name):
     if not t.is_cuda:

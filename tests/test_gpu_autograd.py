@@ -897,3 +897,67 @@ def test_fused_training_functions_on_a_graph_without_edges(pkg):
     assert len(prods) == 13 and all(float(p.abs().sum()) == 0.0 for p in prods)
     grads = torch.autograd.grad(sum(p.sum() for p in prods), nodes, allow_unused=True)
     assert all(g is None or float(g.abs().max()) == 0.0 for g in grads)
+
+
+@pytest.mark.parametrize("B,N,n,n_rbf,degree", [(1, 1, 4, 4, 1), (2, 65, 8, 12, 3), (3, 64, 32, 16, 5), (1, 700, 128, 128, 4)])
+def test_painn_layers_of_values_and_tangents(pkg, B, N, n, n_rbf, degree):
+    """Message and Update as the fused functions run them under differentiation: values, forward-mode tangents, the gradients
+    of a function of both for every input and parameter, and (values alone) the gradients without tangents, against the
+    oracle's layers in float64.  Sizes around the pieces of the kernels: one node, a node past a piece of 64, rows of one lane
+    up to a wave, one and several pieces of the group norm's statistics, products of 4 and of 1024 gradient rows.  Tolerance: a gradient
+    here is a chain of at most ten sums of up to 700 terms, 10 sqrt(700) 2^-24 = 1.6e-5 of the largest entry."""
+    painn = importlib.import_module("learned-dynamics_amd.painn")
+    gl = importlib.import_module("learned-dynamics_amd.graph_layers")
+    diff = importlib.import_module("learned-dynamics_amd.differentiable")
+    torch.manual_seed(0x947 + n)
+    gen = torch.Generator().manual_seed(7 + N)
+    r0 = 5.0
+    rnd = lambda *shape: torch.randn(*shape, generator=gen)
+    src = torch.arange(B * N).repeat_interleave(degree)
+    if N > 1:
+        src = src[src % N != 1]                                          # (a node without edges)
+    dst = (src // N) * N + torch.randint(0, N, (len(src),), generator=gen)
+    msg, upd = painn.Message(r0, n, n_rbf).cuda(), painn.Update(n).cuda()
+    with torch.no_grad():
+        upd.gn.gamma.normal_(); upd.gn.beta.normal_()
+    graph = gl.Graph(src.cuda(), dst.cuda(), None, B, N)
+    x = [rnd(B, N, n), rnd(B, N, n, 3), 2 * rnd(len(src), 3)]
+    t = [rnd(*a.shape) for a in x]
+    c = [rnd(B, N, n), rnd(B, N, n, 3), rnd(B, N, n), rnd(B, N, n, 3)]
+
+    def layers(msg_f, upd_f):
+        def f(xa, xv, r):
+            da, dv = msg_f(xa, xv, r)
+            return upd_f(xa + da, xv + dv)
+        return f
+
+    wd, wa, wu_mlp = _mlp_w(msg.mlp_dist), _mlp_w(msg.mlp_actv), _mlp_w(upd.mlp)
+    copy = lambda p: p.detach().cpu().double().requires_grad_(True)
+    wu = {"W_l": copy(upd.lin_l.W), "W_r": copy(upd.lin_r.W), "W_v": copy(upd.lin_v.W), "mlp": wu_mlp,
+          "gn_gamma": copy(upd.gn.gamma), "gn_beta": copy(upd.gn.beta)}
+    params_o = []
+    for w in (wd, wa, wu_mlp):
+        for k in ("W1", "b1", "W2", "b2", "W3", "b3"):
+            params_o.append(w[k].requires_grad_(True))
+    params_o += [wu[k] for k in ("W_l", "W_r", "W_v", "gn_gamma", "gn_beta")]
+    params_d = [p for m in (msg.mlp_dist, msg.mlp_actv, upd.mlp) for k in (0, 2, 4) for p in (m.layers[k].weight, m.layers[k].bias)]
+    params_d += [upd.lin_l.W, upd.lin_r.W, upd.lin_v.W, upd.gn.gamma, upd.gn.beta]
+    f_d = layers(lambda xa, xv, r: msg(graph, xa, xv, r), upd)
+    f_o = layers(lambda xa, xv, r: OL.painn_message(src, dst, B, N, xa, xv, r, wd, wa, r0, n, n_rbf),
+                 lambda xa, xv: OL.painn_update(xa, xv, wu, n))
+    x_d, x_o = [a.cuda().requires_grad_() for a in x], [a.double().requires_grad_() for a in x]
+    t_d, t_o = tuple(a.cuda() for a in t), tuple(a.double() for a in t)
+    value_d, tangent_d = diff.jvp(f_d, tuple(x_d), t_d)
+    value_o, tangent_o = torch.autograd.functional.jvp(f_o, tuple(x_o), t_o, create_graph=True)
+    for k, name in enumerate(("a", "v")):
+        _close(value_d[k], value_o[k], f"value {name}", 1.6e-5)
+        _close(tangent_d[k], tangent_o[k], f"tangent {name}", 1.6e-5)
+    total = lambda vs, to: sum((v * to(w)).sum() for v, w in zip(vs, c))
+    g_d = torch.autograd.grad(total((*value_d, *tangent_d), lambda w: w.cuda()), x_d + params_d)
+    g_o = torch.autograd.grad(total((*value_o, *tangent_o), lambda w: w.double()), x_o + params_o)
+    for k, (a, b) in enumerate(zip(g_d, g_o)):
+        _close(a, b, f"gradient {k} through value and tangent", 1.6e-5)
+    g_d = torch.autograd.grad(total(f_d(*x_d), lambda w: w.cuda()), x_d + params_d)
+    g_o = torch.autograd.grad(total(f_o(*x_o), lambda w: w.double()), x_o + params_o)
+    for k, (a, b) in enumerate(zip(g_d, g_o)):
+        _close(a, b, f"gradient {k}", 1.6e-5)
