@@ -569,6 +569,28 @@ int mg_bee_edge_filters_bwd(const float* enc, const float* rh, const float* g_v,
  * n floats, 16-byte aligned.  The reference leaves these derivatives to autograd's elementwise formulas. */
 int mg_silu_order(const float* z, const float* mul, long n, int order, float* out, mg_stream_t stream);
 
+/* Gradients of mg_painn_table_message_sliced for actv, v and the grid (edge vectors not differentiated): g_v (n_nodes, n, 3),
+ * g_a (n_nodes, n) are the gradients of its outputs.  n a multiple of 16 up to 256, table_rows as there
+ * (mg_painn_grid_grad_supported: 0 / 1).  One workspace serves both; calls on one stream may share it. */
+int mg_painn_grid_grad_supported(int table_rows, int n);
+int mg_painn_grid_grad_workspace_bytes(int table_rows, int n, long n_edges, size_t* bytes /* host */);
+/* d_actv (n_nodes, 4n) and d_v (n_nodes, n, 3), either may be NULL.  row_ptr / order: the edges that read each node (order NULL:
+ * the positions themselves), src: every edge's source; node_order: the order in which nodes are taken, or NULL. */
+int mg_painn_grid_node_grad(const int* row_ptr, const int* order, const int* src, const int* node_order, int n_nodes, long n_edges,
+                            const float* r_ij, const float* table, int table_rows, float period, float epsilon, const float* g_v,
+                            const float* g_a, const float* actv, const float* v, int n, void* workspace, float* d_actv, float* d_v,
+                            mg_stream_t stream);
+/* row[e]: the grid row below an edge's length */
+int mg_painn_grid_rows(const float* r_ij, long n_edges, int table_rows, float period, int* row, mg_stream_t stream);
+/* d_table (table_rows, 4n).  order / bucket_ptr: the edges sorted by mg_painn_grid_rows; actv_sliced as in
+ * mg_painn_table_message_sliced. */
+int mg_painn_grid_table_grad(const int* order, const int* bucket_ptr, const int* src, const int* dst, int n_nodes, long n_edges,
+                             const float* r_ij, int table_rows, float period, float epsilon, const float* g_v, const float* g_a,
+                             const float* actv_sliced, const float* v, int n, void* workspace, float* d_table, mg_stream_t stream);
+/* order: the positions of keys (0 .. key_limit - 1) in the order of a stable sort; sorted_keys: the keys in that order. */
+int mg_sort_by_key_workspace_bytes(long count, size_t* bytes /* host */);
+int mg_sort_by_key(const int* keys, long count, int key_limit, void* workspace, int* order, int* sorted_keys, mg_stream_t stream);
+
 /* The PaiNN layers under differentiation (archs/meanflow_painn8.py:25-100; the meanflow loss, :274-296): the passes between the
  * linear maps, forward and adjoint.  dual != 0: every array holds `rows` rows of values and then `rows` rows of forward-mode
  * tangents, and both halves are read and written in one pass; dual == 0: values alone.  n is a multiple of 4, arrays of rows are

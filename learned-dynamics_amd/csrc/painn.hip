@@ -14,6 +14,7 @@
 // narrower than the wave the spare lanes take the next edges of the same node and
 // are folded with xor-shuffles.  Rows are summed in edge order: no atomics.
 #include "common.hpp"
+#include "lane_sums.hpp"
 
 namespace mg {
 namespace {
@@ -229,8 +230,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TABLE 
 // instructions before).  The grid in LDS carries three extra rows (copies of rows 0..2) behind the last one, so the
 // four rows of an edge are always consecutive: one address per edge, the rest are immediates.
 // LDS rows are padded to 68 floats so that the rows different edges read start in different banks.
-constexpr int kSliceChan = 16, kSliceCols = 4 * kSliceChan, kSliceRowF = kSliceCols + 4, kSliceMaxRows = 512;
-constexpr int kSliceExtraRows = 3;
 
 // rec[2e] = (float offset of the first grid row in LDS as int bits, w0, w1, w2), rec[2e+1] = (w3, ux, uy, uz):
 // grid rows i-1 .. i+2 with i = floor(|r| / h), 4-point Lagrange weights at t = |r| / h - i, u = r / sqrt(eps + |r|^2)
@@ -250,25 +249,6 @@ __global__ void __launch_bounds__(256) painn_edge_records_kernel(const float* __
     const float inv = 1.0f / sqrtf(epsilon + r2);
     rec[2 * e] = make_float4(__int_as_float(first * kSliceRowF), w0, w1, w2);
     rec[2 * e + 1] = make_float4(w3, rx * inv, ry * inv, rz * inv);
-}
-
-// Sum of 16 per-lane values over the 16 lanes that share (lane & 3), leaving value s of the 16 in the lane with
-// (lane >> 2) == s: each step pairs the registers, exchanges the halves two lanes do not keep and adds, so the whole
-// reduction is 15 additions instead of 16 x 4.  Lane halves (xor 32) and odd / even rows of 16 lanes (xor 16) are
-// exchanged by the swap instructions, lanes 8 and 4 apart by LDS-crossbar swizzles.
-__device__ __forceinline__ void swap_add32(float& a, const float b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    a = __uint_as_float(r[0]) + __uint_as_float(r[1]);        // lanes 0..31: a over both halves; 32..63: b
-}
-__device__ __forceinline__ void swap_add16(float& a, const float b) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    a = __uint_as_float(r[0]) + __uint_as_float(r[1]);        // even rows of 16 lanes: a; odd rows: b
-}
-template <int XOR>
-__device__ __forceinline__ void swizzle_add(float& a, const float b, bool upper) {
-    const float keep = upper ? b : a, send = upper ? a : b;
-    constexpr int pattern = (XOR << 10) | 0x1f;               // lane' = lane ^ XOR inside each group of 32
-    a = keep + __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(send), pattern));
 }
 
 __global__ void __launch_bounds__(1024) painn_table_message_lds_kernel(
@@ -347,16 +327,8 @@ __global__ void __launch_bounds__(1024) painn_table_message_lds_kernel(
             }
             j = j_next; ra = na; rb = nb;
         }
-        // 16 sums over the 16 edge slots of the wave: value index sub = bit2 + 2 bit3 + 4 bit4 + 8 bit5 of the lane id
-#pragma unroll
-        for (int k = 0; k < 8; k++) swap_add32(acc[k], acc[k + 8]);          // registers 0..7: value k + 8 bit5
-#pragma unroll
-        for (int k = 0; k < 4; k++) swap_add16(acc[k], acc[k + 4]);          // registers 0..3: value k + 4 bit4 + 8 bit5
-#pragma unroll
-        for (int k = 0; k < 2; k++) swizzle_add<8>(acc[k], acc[k + 2], (lane & 8) != 0);
-        swizzle_add<4>(acc[0], acc[1], (lane & 4) != 0);
         const long o = node * n + o_lane;
-        float sum = acc[0];
+        float sum = sum_over_slots(acc, lane);
         float* outp = is_a ? out_a + o + (sub - 12) : out_v + o * 3 + sub;
         const float* resp = is_a ? (res_a ? res_a + o + (sub - 12) : nullptr) : (res_v ? res_v + o * 3 + sub : nullptr);
         if (resp) sum += *resp;

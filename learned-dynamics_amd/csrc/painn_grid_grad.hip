@@ -1,0 +1,468 @@
+// Gradients of the PaiNN message whose filter is interpolated from its grid (painn.hip, painn_table_message_lds_kernel), for
+// edge vectors that are not differentiated.  With f the filter of an edge (4 blocks of n columns), a and v the rows of its
+// destination, u its direction, and (g, ga) the gradient rows of its source:
+//   d_actv[r] = (v . M0, v . M1, S2, S3),  d_v[r] = a0 M0 + a1 M1   with the sums over the edges that read row r
+//   M0 = sum f0 g,  M1 = sum f1 (u x g),  S2 = sum f2 (u . g),  S3 = sum f3 ga
+//   d_grid[i, k] = sum over edges and taps of w (dp_k a_k),  dp = (g . v, v . (u x g), u . g, ga)
+// The first line needs only the 8 sums per channel: a and v of the row come in once at the end, an edge reads its source's g and
+// ga (2 KB at n = 128; the pass it replaces also read four grid rows from the caches, 8 KB, and wrote the edge's 2 KB of
+// d_filter).  The second takes the edges in the order of their grid rows, so that the 4 taps x 4 blocks of a row are sums in
+// registers, and forms d_filter itself from the node rows: no per-edge array is written or read (3.3 GB each way at 1.6 M
+// edges).  16384 nodes, 1.6 M edges, n = 128: see the figures at the two kernels.
+#include "common.hpp"
+#include "lane_sums.hpp"
+
+namespace mg {
+namespace {
+
+__device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+__device__ __forceinline__ void st4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
+
+// |r| / h and 1 / sqrt(eps + |r|^2).  (The fused multiply-adds are spelled out: every kernel here that puts an edge into a grid
+// row must find the same one.)
+struct EdgePlace { float u, inv; };
+__device__ __forceinline__ EdgePlace place(float x, float y, float z, float inv_h, float eps) {
+    const float r2 = fmaf(x, x, fmaf(y, y, z * z));
+    return {sqrtf(r2) * inv_h, 1.0f / sqrtf(eps + r2)};
+}
+__device__ __forceinline__ void lagrange(float t, float (&w)[4]) {
+    const float tp = t + 1.0f, tm = t - 1.0f, tq = t - 2.0f;
+    w[0] = -(1.0f / 6.0f) * t * tm * tq;
+    w[1] = 0.5f * tp * tm * tq;
+    w[2] = -0.5f * tp * t * tq;
+    w[3] = (1.0f / 6.0f) * tp * t * tm;
+}
+
+// ------------------------------------------------------------------------------------------------ records
+// Per position of the order by destination: (float offset of the first grid row in LDS as int bits, w0, w1, w2), (w3, u), and
+// the source.
+__global__ void __launch_bounds__(256) node_records_kernel(const float* __restrict__ r_ij, const int* __restrict__ order,
+                                                           const int* __restrict__ src, long E, int mask, float inv_h, float eps,
+                                                           float4* __restrict__ rec, int* __restrict__ from) {
+    const long p = (long)blockIdx.x * 256 + threadIdx.x;
+    if (p >= E) return;
+    const long e = order ? min(max((long)order[p], 0L), E - 1) : p;
+    const float x = r_ij[3 * e], y = r_ij[3 * e + 1], z = r_ij[3 * e + 2];
+    const EdgePlace q = place(x, y, z, inv_h, eps);
+    const float fl = floorf(q.u);
+    float w[4];
+    lagrange(q.u - fl, w);
+    const int first = ((int)fl - 1) & mask;
+    rec[2 * p] = make_float4(__int_as_float(first * kSliceRowF), w[0], w[1], w[2]);
+    rec[2 * p + 1] = make_float4(w[3], x * q.inv, y * q.inv, z * q.inv);
+    from[p] = src[e];
+}
+// Per position of the order by grid row: (source, destination as int bits, t, ux), (uy, uz, 0, 0)
+__global__ void __launch_bounds__(256) row_records_kernel(const float* __restrict__ r_ij, const int* __restrict__ order,
+                                                          const int* __restrict__ src, const int* __restrict__ dst, long E,
+                                                          float inv_h, float eps, float4* __restrict__ rec) {
+    const long p = (long)blockIdx.x * 256 + threadIdx.x;
+    if (p >= E) return;
+    const long e = min(max((long)order[p], 0L), E - 1);
+    const float x = r_ij[3 * e], y = r_ij[3 * e + 1], z = r_ij[3 * e + 2];
+    const EdgePlace q = place(x, y, z, inv_h, eps);
+    rec[2 * p] = make_float4(__int_as_float(src[e]), __int_as_float(dst[e]), q.u - floorf(q.u), x * q.inv);
+    rec[2 * p + 1] = make_float4(y * q.inv, z * q.inv, 0.f, 0.f);
+}
+__global__ void __launch_bounds__(256) grid_row_kernel(const float* __restrict__ r_ij, long E, int mask, float inv_h, float eps,
+                                                       int* __restrict__ row) {
+    const long e = (long)blockIdx.x * 256 + threadIdx.x;
+    if (e < E) row[e] = (int)floorf(place(r_ij[3 * e], r_ij[3 * e + 1], r_ij[3 * e + 2], inv_h, eps).u) & mask;
+}
+
+// ------------------------------------------------------------------------------------------------ gradients of actv and v
+// The mapping of painn_table_message_lds_kernel: a workgroup holds one slice of 16 channels of the grid in LDS, a wave takes 16
+// edges of its node per step, 4 lanes x 4 channels each.  Bound by vector issue, like that kernel.
+__global__ void __launch_bounds__(1024) grid_node_grad_kernel(
+    const int* __restrict__ row_ptr, const int* __restrict__ from, const int* __restrict__ node_order, long n_nodes, long E,
+    const float4* __restrict__ rec, const float* __restrict__ table, int tab_rows, const float* __restrict__ g_v,
+    const float* __restrict__ g_a, const float* __restrict__ actv, const float* __restrict__ v, int n,
+    float* __restrict__ d_actv, float* __restrict__ d_v) {
+    extern __shared__ float tab[];                            // (tab_rows + 3) x kSliceRowF
+    const int n_slices = n / kSliceChan;
+    const int slice = blockIdx.x % n_slices;
+    const int group = blockIdx.x / n_slices, groups = gridDim.x / n_slices;
+    for (int q = threadIdx.x; q < (tab_rows + kSliceExtraRows) * (kSliceCols / 4); q += blockDim.x) {
+        const int row = q / (kSliceCols / 4), piece = q % (kSliceCols / 4), k = piece / 4, c4 = piece % 4;
+        st4(tab + row * kSliceRowF + 4 * piece,
+            ld4(table + (long)(row & (tab_rows - 1)) * 4 * n + k * n + slice * kSliceChan + 4 * c4));
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, waves = blockDim.x / kWave;
+    const int l4 = lane & 3, sub = lane >> 2;
+    constexpr int kPerIter = kWave / 4;
+    const float* gv_base = g_v + (slice * kSliceChan + 4 * l4) * 3;
+    const float* ga_base = g_a + slice * kSliceChan + 4 * l4;
+    const unsigned v_stride = 3u * (unsigned)n, a_stride = (unsigned)n;
+    const float* tab_l = tab + 4 * l4;
+    for (long slot = (long)group * waves + wave; slot < n_nodes; slot += (long)groups * waves) {
+        const long node = node_order ? node_order[slot] : slot;
+        const int lo = max(row_ptr[node], 0), hi = min(row_ptr[node + 1], (int)E);
+        // value 4 c + q of channel c: (M0, S2) and (M1, S3)
+        float A[16], B[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) { A[k] = 0.f; B[k] = 0.f; }
+        int e = lo + sub;
+        unsigned j = 0;
+        float4 ra = make_float4(0.f, 0.f, 0.f, 0.f), rb = ra;
+        if (e < hi) { j = (unsigned)from[e]; ra = rec[2 * (long)e]; rb = rec[2 * (long)e + 1]; }
+        while (e < hi) {
+            const float* gv = gv_base + (long)j * v_stride;
+            const float4 g0 = ld4(gv), g1 = ld4(gv + 4), g2 = ld4(gv + 8), ga = ld4(ga_base + (long)j * a_stride);
+            e += kPerIter;
+            unsigned j_next = 0;
+            float4 na = ra, nb = rb;
+            if (e < hi) { j_next = (unsigned)from[e]; na = rec[2 * (long)e]; nb = rec[2 * (long)e + 1]; }
+            const float* tp = tab_l + __float_as_int(ra.x);
+            const float w0 = ra.y, w1 = ra.z, w2 = ra.w, w3 = rb.x, ux = rb.y, uy = rb.z, uz = rb.w;
+            float f[4][4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float4 t0 = ld4(tp + k * kSliceChan), t1 = ld4(tp + kSliceRowF + k * kSliceChan),
+                             t2 = ld4(tp + 2 * kSliceRowF + k * kSliceChan), t3 = ld4(tp + 3 * kSliceRowF + k * kSliceChan);
+                f[k][0] = w0 * t0.x + w1 * t1.x + w2 * t2.x + w3 * t3.x;
+                f[k][1] = w0 * t0.y + w1 * t1.y + w2 * t2.y + w3 * t3.y;
+                f[k][2] = w0 * t0.z + w1 * t1.z + w2 * t2.z + w3 * t3.z;
+                f[k][3] = w0 * t0.w + w1 * t1.w + w2 * t2.w + w3 * t3.w;
+            }
+            const float gg[12] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w, g2.x, g2.y, g2.z, g2.w};
+            const float gs[4] = {ga.x, ga.y, ga.z, ga.w};
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const float x = gg[3 * c], y = gg[3 * c + 1], z = gg[3 * c + 2];
+                A[4 * c + 0] = fmaf(f[0][c], x, A[4 * c + 0]);
+                A[4 * c + 1] = fmaf(f[0][c], y, A[4 * c + 1]);
+                A[4 * c + 2] = fmaf(f[0][c], z, A[4 * c + 2]);
+                A[4 * c + 3] = fmaf(f[2][c], ux * x + uy * y + uz * z, A[4 * c + 3]);
+                B[4 * c + 0] = fmaf(f[1][c], uy * z - uz * y, B[4 * c + 0]);                 // u x g
+                B[4 * c + 1] = fmaf(f[1][c], uz * x - ux * z, B[4 * c + 1]);
+                B[4 * c + 2] = fmaf(f[1][c], ux * y - uy * x, B[4 * c + 2]);
+                B[4 * c + 3] = fmaf(f[3][c], gs[c], B[4 * c + 3]);
+            }
+            j = j_next; ra = na; rb = nb;
+        }
+        const float sA = sum_over_slots(A, lane), sB = sum_over_slots(B, lane);
+        const int c = sub >> 2, q = sub & 3;
+        const long ch = slice * kSliceChan + 4 * l4 + c, row4 = node * 4L * n + ch;
+        const float vq = q < 3 ? v[(node * n + ch) * 3 + q] : 0.f;
+        float s0 = vq * sA, s1 = vq * sB;                     // v . M0, v . M1: over the lanes q = 0..2 of the channel
+        s0 += __shfl_xor(s0, 4); s1 += __shfl_xor(s1, 4);
+        s0 += __shfl_xor(s0, 8); s1 += __shfl_xor(s1, 8);
+        if (d_v && q < 3) d_v[(node * n + ch) * 3 + q] = actv[row4] * sA + actv[row4 + n] * sB;
+        if (d_actv) {
+            if (q == 3) { d_actv[row4 + 2 * n] = sA; d_actv[row4 + 3 * n] = sB; }
+            else if (q < 2) d_actv[row4 + q * n] = q ? s1 : s0;
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------ gradient of the grid
+// part[((row splits + s) 4 + j) 4n + k n + c]: piece s of the edges of a grid row, in order; a wave takes 16 edges per step as
+// above, its 64 sums per lane are added over the slots at the end and over the 4 waves in wave order.  Slices are the fastest
+// block index (one slice per XCD at n = 128), pieces the slowest: the blocks that run together read the rows of the same part
+// of the nodes.  Bound by those reads (11 x 16 bytes per lane and edge against 64 multiply-adds).
+__global__ void __launch_bounds__(256) grid_row_grad_kernel(const int* __restrict__ bucket_ptr, const float4* __restrict__ rec,
+                                                            long E, int rows, int splits, long n_nodes,
+                                                            const float* __restrict__ actv_s, const float* __restrict__ v,
+                                                            const float* __restrict__ g_v, const float* __restrict__ g_a, int n,
+                                                            float* __restrict__ part) {
+    __shared__ float fold[4][4][kWave];
+    const int n_slices = n / kSliceChan;
+    const int slice = blockIdx.x % n_slices, rest = blockIdx.x / n_slices;
+    const int row = rest % rows, s = rest / rows;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int l4 = lane & 3, sub = lane >> 2;
+    const long b_lo = max((long)bucket_ptr[row], 0L), b_hi = min((long)bucket_ptr[row + 1], E), len = b_hi - b_lo;
+    const long lo = b_lo + len * s / splits, hi = b_lo + len * (s + 1) / splits;
+    const float* a_base = actv_s + slice * kSliceCols + 4 * l4;
+    const float* v_base = v + (slice * kSliceChan + 4 * l4) * 3;
+    const float* gv_base = g_v + (slice * kSliceChan + 4 * l4) * 3;
+    const float* ga_base = g_a + slice * kSliceChan + 4 * l4;
+    float acc[4][16];                                         // tap j; value 4 k + c
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int k = 0; k < 16; k++) acc[j][k] = 0.f;
+    long e = lo + 16 * wave + sub;
+    float4 ra = make_float4(0.f, 0.f, 0.f, 0.f), rb = ra;
+    if (e < hi) { ra = rec[2 * e]; rb = rec[2 * e + 1]; }
+    while (e < hi) {
+        const long from = min(max((long)__float_as_int(ra.x), 0L), n_nodes - 1), to = min(max((long)__float_as_int(ra.y), 0L), n_nodes - 1);
+        const float* ap = a_base + to * 4 * n;
+        const float* vp = v_base + to * 3 * n;
+        const float* gp = gv_base + from * 3 * n;
+        float4 a[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) a[k] = ld4(ap + k * kSliceChan);
+        const float4 v0 = ld4(vp), v1 = ld4(vp + 4), v2 = ld4(vp + 8);
+        const float4 g0 = ld4(gp), g1 = ld4(gp + 4), g2 = ld4(gp + 8), ga = ld4(ga_base + from * n);
+        e += 64;
+        float4 na = ra, nb = rb;
+        if (e < hi) { na = rec[2 * e]; nb = rec[2 * e + 1]; }
+        const float ux = ra.w, uy = rb.x, uz = rb.y;
+        float w[4];
+        lagrange(ra.z, w);
+        const float vv[12] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w, v2.x, v2.y, v2.z, v2.w};
+        const float gg[12] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w, g2.x, g2.y, g2.z, g2.w};
+        const float gs[4] = {ga.x, ga.y, ga.z, ga.w};
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const float x = gg[3 * c], y = gg[3 * c + 1], z = gg[3 * c + 2];
+            const float vx = vv[3 * c], vy = vv[3 * c + 1], vz = vv[3 * c + 2];
+            const float av[4] = {c == 0 ? a[0].x : c == 1 ? a[0].y : c == 2 ? a[0].z : a[0].w,
+                                 c == 0 ? a[1].x : c == 1 ? a[1].y : c == 2 ? a[1].z : a[1].w,
+                                 c == 0 ? a[2].x : c == 1 ? a[2].y : c == 2 ? a[2].z : a[2].w,
+                                 c == 0 ? a[3].x : c == 1 ? a[3].y : c == 2 ? a[3].z : a[3].w};
+            const float d[4] = {(x * vx + y * vy + z * vz) * av[0],
+                                ((uy * z - uz * y) * vx + (uz * x - ux * z) * vy + (ux * y - uy * x) * vz) * av[1],
+                                (ux * x + uy * y + uz * z) * av[2], gs[c] * av[3]};
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[j][4 * k + c] = fmaf(w[j], d[k], acc[j][4 * k + c]);
+        }
+        ra = na; rb = nb;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) fold[wave][j][lane] = sum_over_slots(acc[j], lane);
+    __syncthreads();
+    // wave j adds tap j over the four waves; value `sub` = 4 k + c of the channel quad l4
+    const float sum = (fold[0][wave][lane] + fold[1][wave][lane]) + (fold[2][wave][lane] + fold[3][wave][lane]);
+    part[(((long)row * splits + s) * 4 + wave) * 4 * n + (sub >> 2) * n + slice * kSliceChan + 4 * l4 + (sub & 3)] = sum;
+}
+
+// d_table[m, :] = the sum over pieces and taps of the parts that touch row m, in this order
+__global__ void __launch_bounds__(256) grid_grad_finish_kernel(const float* __restrict__ part, int rows, int cols, int splits,
+                                                               float* __restrict__ d_table) {
+    const int quads = cols >> 2;
+    const long t = (long)blockIdx.x * 256 + threadIdx.x;
+    const long m = t / quads;
+    if (m >= rows) return;
+    const int c = (int)(t - m * quads) * 4;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int j = 0; j < 4; j++) {
+        const long row = (m + 1 - j) & (rows - 1);
+        for (int s = 0; s < splits; s++) {
+            const float4 p = ld4(part + ((row * splits + s) * 4 + j) * (long)cols + c);
+            acc.x += p.x; acc.y += p.y; acc.z += p.z; acc.w += p.w;
+        }
+    }
+    st4(d_table + m * cols + c, acc);
+}
+
+// ------------------------------------------------------------------------------------------------ stable sort by small keys
+// One pass of a stable radix sort on 9 bits: counts per (digit, chunk of 4096), their prefix sums per digit, and the scatter,
+// in which a wave ranks 64 elements at a time by comparing digits across lanes.  (torch.sort on these keys takes 10 launches:
+// 150 us for 1.6 M edges, 90 for 90 000; this takes 3.)
+constexpr int kDigits = 512, kDigitBits = 9, kSortChunk = 4096;
+__device__ __forceinline__ int digit_of(const int* keys, long i, int shift) { return (keys[i] >> shift) & (kDigits - 1); }
+
+__global__ void __launch_bounds__(256) sort_count_kernel(const int* __restrict__ keys, long n, int shift, int chunks,
+                                                         int* __restrict__ counts) {
+    __shared__ int hist[kDigits];
+    for (int d = threadIdx.x; d < kDigits; d += 256) hist[d] = 0;
+    __syncthreads();
+    const long lo = (long)blockIdx.x * kSortChunk, hi = min(lo + kSortChunk, n);
+    for (long i = lo + threadIdx.x; i < hi; i += 256) atomicAdd(&hist[digit_of(keys, i, shift)], 1);
+    __syncthreads();
+    for (int d = threadIdx.x; d < kDigits; d += 256) counts[(long)d * chunks + blockIdx.x] = hist[d];
+}
+// counts[d] -> exclusive prefix sums over the chunks; totals[d]
+__global__ void __launch_bounds__(64) sort_prefix_kernel(int* __restrict__ counts, int chunks, int* __restrict__ totals) {
+    int* row = counts + (long)blockIdx.x * chunks;
+    int base = 0;
+    for (int c0 = 0; c0 < chunks; c0 += 64) {
+        const int c = c0 + threadIdx.x;
+        const int own = c < chunks ? row[c] : 0;
+        int sum = own;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int up = __shfl_up(sum, d);
+            if ((int)threadIdx.x >= d) sum += up;
+        }
+        if (c < chunks) row[c] = base + sum - own;
+        base += __shfl(sum, 63);
+    }
+    if (threadIdx.x == 0) totals[blockIdx.x] = base;
+}
+__global__ void __launch_bounds__(256) sort_scatter_kernel(const int* __restrict__ keys, const int* __restrict__ values, long n,
+                                                           int shift, int chunks, const int* __restrict__ counts,
+                                                           const int* __restrict__ totals, int* __restrict__ keys_out,
+                                                           int* __restrict__ values_out) {
+    __shared__ int at[4][kDigits];                            // next output position per wave and digit
+    __shared__ int wave_sum[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // exclusive prefix sums of the totals: two digits per thread
+    {
+        const int a = totals[2 * tid], b = totals[2 * tid + 1];
+        int sum = a + b;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int up = __shfl_up(sum, d);
+            if (lane >= d) sum += up;
+        }
+        if (lane == 63) wave_sum[wave] = sum;
+        __syncthreads();
+        int before = sum - a - b;
+        for (int w = 0; w < wave; w++) before += wave_sum[w];
+        at[0][2 * tid] = before + counts[(long)(2 * tid) * chunks + blockIdx.x];
+        at[0][2 * tid + 1] = before + a + counts[(long)(2 * tid + 1) * chunks + blockIdx.x];
+        for (int w = 1; w < 4; w++) { at[w][2 * tid] = 0; at[w][2 * tid + 1] = 0; }
+    }
+    __syncthreads();
+    const long lo = (long)blockIdx.x * kSortChunk + (long)wave * (kSortChunk / 4);
+    const long hi = min(min(lo + kSortChunk / 4, ((long)blockIdx.x + 1) * kSortChunk), n);
+    // how many of each digit the waves before this one hold
+    if (wave < 3)
+        for (long i = lo + lane; i < hi; i += 64) {
+            const int d = digit_of(keys, i, shift);
+            for (int w = wave + 1; w < 4; w++) atomicAdd(&at[w][d], 1);
+        }
+    __syncthreads();
+    for (int d = tid; d < kDigits; d += 256)
+        for (int w = 1; w < 4; w++) at[w][d] += at[0][d];
+    __syncthreads();
+    for (long i0 = lo; i0 < hi; i0 += 64) {
+        const long i = i0 + lane;
+        const bool live = i < hi;
+        const int key = live ? keys[i] : 0;
+        const int d = (key >> shift) & (kDigits - 1);
+        unsigned long long same = __ballot(live);
+#pragma unroll
+        for (int b = 0; b < kDigitBits; b++) {
+            const unsigned long long m = __ballot((d >> b) & 1);
+            same &= ((d >> b) & 1) ? m : ~m;
+        }
+        const int rank = __popcll(same & ((1ull << lane) - 1ull));
+        int pos = 0;
+        if (live) pos = at[wave][d] + rank;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (live && rank == 0) at[wave][d] = pos + __popcll(same);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (live) {
+            values_out[pos] = values ? values[i] : (int)i;
+            if (keys_out) keys_out[pos] = key;
+        }
+    }
+}
+
+int splits_of(int rows, long E) {
+    // pieces of about 768 edges: 12 steps of the 4 waves, against which adding 64 sums over the slots is a fifth
+    long s = ceil_div(E, 768L * rows);
+    return (int)(s < 1 ? 1 : (s > 16 ? 16 : s));
+}
+
+}  // namespace
+}  // namespace mg
+
+using namespace mg;
+
+extern "C" {
+
+int mg_painn_grid_grad_supported(int table_rows, int n) {
+    return n >= kSliceChan && n % kSliceChan == 0 && n <= 256 && table_rows >= 4 && table_rows <= kSliceMaxRows &&
+                   (table_rows & (table_rows - 1)) == 0
+               ? 1
+               : 0;
+}
+
+int mg_painn_grid_grad_workspace_bytes(int table_rows, int n, long n_edges, size_t* bytes) {
+    MG_REQUIRE(bytes && n_edges >= 0 && mg_painn_grid_grad_supported(table_rows, n), "mg_painn_grid_grad_workspace_bytes: bad argument");
+    const size_t by_node = (size_t)n_edges * 36, by_row = (size_t)n_edges * 32 + (size_t)table_rows * splits_of(table_rows, n_edges) * 16 * n * sizeof(float);
+    *bytes = (by_node > by_row ? by_node : by_row) + 32;
+    return MG_OK;
+}
+
+int mg_painn_grid_node_grad(const int* row_ptr, const int* order, const int* src, const int* node_order, int n_nodes, long n_edges,
+                            const float* r_ij, const float* table, int table_rows, float period, float epsilon, const float* g_v,
+                            const float* g_a, const float* actv, const float* v, int n, void* workspace, float* d_actv, float* d_v,
+                            mg_stream_t stream) {
+    MG_REQUIRE(n_nodes >= 0 && n_edges >= 0 && n_edges < (1L << 31) && period > 0.f && mg_painn_grid_grad_supported(table_rows, n),
+               "mg_painn_grid_node_grad: bad argument");
+    if (n_nodes == 0) return MG_OK;
+    MG_REQUIRE(row_ptr && table && g_v && g_a && actv && v && workspace && (n_edges == 0 || (src && r_ij)) && aligned16(table) &&
+                   aligned16(g_v) && aligned16(g_a),
+               "mg_painn_grid_node_grad: null or unaligned pointer");
+    hipStream_t st = (hipStream_t)stream;
+    float4* rec = reinterpret_cast<float4*>((reinterpret_cast<uintptr_t>(workspace) + 15) & ~uintptr_t(15));
+    int* from = reinterpret_cast<int*>(rec + 2 * n_edges);
+    if (n_edges > 0)
+        hipLaunchKernelGGL(node_records_kernel, dim3((unsigned)ceil_div(n_edges, 256)), dim3(256), 0, st, r_ij, order, src, n_edges,
+                           table_rows - 1, (float)table_rows / period, epsilon, rec, from);
+    const int n_slices = n / kSliceChan;
+    MG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(grid_node_grad_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (kSliceMaxRows + kSliceExtraRows) * kSliceRowF * (int)sizeof(float)));
+    long groups = ceil_div(256, n_slices);                    // one workgroup per CU
+    const long max_groups = ceil_div(n_nodes, 16);
+    if (groups > max_groups) groups = max_groups;
+    hipLaunchKernelGGL(grid_node_grad_kernel, dim3((unsigned)(groups * n_slices)), dim3(1024),
+                       (size_t)(table_rows + kSliceExtraRows) * kSliceRowF * sizeof(float), st, row_ptr, from, node_order,
+                       (long)n_nodes, n_edges, rec, table, table_rows, g_v, g_a, actv, v, n, d_actv, d_v);
+    return check_launch("mg_painn_grid_node_grad");
+}
+
+int mg_painn_grid_rows(const float* r_ij, long n_edges, int table_rows, float period, int* row, mg_stream_t stream) {
+    MG_REQUIRE(n_edges >= 0 && period > 0.f && table_rows >= 4 && (table_rows & (table_rows - 1)) == 0, "mg_painn_grid_rows: bad argument");
+    if (n_edges == 0) return MG_OK;
+    MG_REQUIRE(r_ij && row, "mg_painn_grid_rows: null pointer");
+    hipLaunchKernelGGL(grid_row_kernel, dim3((unsigned)ceil_div(n_edges, 256)), dim3(256), 0, (hipStream_t)stream, r_ij, n_edges,
+                       table_rows - 1, (float)table_rows / period, 1.0f, row);
+    return check_launch("mg_painn_grid_rows");
+}
+
+int mg_painn_grid_table_grad(const int* order, const int* bucket_ptr, const int* src, const int* dst, int n_nodes, long n_edges,
+                             const float* r_ij, int table_rows, float period, float epsilon, const float* g_v, const float* g_a,
+                             const float* actv_sliced, const float* v, int n, void* workspace, float* d_table, mg_stream_t stream) {
+    MG_REQUIRE(n_nodes >= 0 && n_edges >= 0 && period > 0.f && mg_painn_grid_grad_supported(table_rows, n) && (n_nodes > 0 || n_edges == 0),
+               "mg_painn_grid_table_grad: bad argument");
+    MG_REQUIRE(bucket_ptr && workspace && d_table && aligned16(d_table), "mg_painn_grid_table_grad: null or unaligned pointer");
+    MG_REQUIRE(n_edges == 0 || (order && src && dst && r_ij && g_v && g_a && actv_sliced && v && aligned16(g_v) && aligned16(g_a) &&
+                                aligned16(actv_sliced) && aligned16(v)),
+               "mg_painn_grid_table_grad: null or unaligned pointer");
+    hipStream_t st = (hipStream_t)stream;
+    float4* rec = reinterpret_cast<float4*>((reinterpret_cast<uintptr_t>(workspace) + 15) & ~uintptr_t(15));
+    float* part = reinterpret_cast<float*>(rec + 2 * n_edges);
+    const int splits = splits_of(table_rows, n_edges), n_slices = n / kSliceChan;
+    if (n_edges > 0)
+        hipLaunchKernelGGL(row_records_kernel, dim3((unsigned)ceil_div(n_edges, 256)), dim3(256), 0, st, r_ij, order, src, dst, n_edges,
+                           (float)table_rows / period, epsilon, rec);
+    hipLaunchKernelGGL(grid_row_grad_kernel, dim3((unsigned)(n_slices * table_rows * splits)), dim3(256), 0, st, bucket_ptr, rec,
+                       n_edges, table_rows, splits, (long)n_nodes, actv_sliced, v, g_v, g_a, n, part);
+    hipLaunchKernelGGL(grid_grad_finish_kernel, dim3((unsigned)ceil_div((long)table_rows * n, 256)), dim3(256), 0, st,
+                       (const float*)part, table_rows, 4 * n, splits, d_table);
+    return check_launch("mg_painn_grid_table_grad");
+}
+
+int mg_sort_by_key_workspace_bytes(long count, size_t* bytes) {
+    MG_REQUIRE(bytes && count >= 0, "mg_sort_by_key_workspace_bytes: bad argument");
+    *bytes = ((size_t)(ceil_div(count, kSortChunk) + 1) * kDigits + 3 * (size_t)count) * sizeof(int);
+    return MG_OK;
+}
+
+int mg_sort_by_key(const int* keys, long count, int key_limit, void* workspace, int* order, int* sorted_keys, mg_stream_t stream) {
+    MG_REQUIRE(count >= 0 && count < (1L << 31) && key_limit >= 1, "mg_sort_by_key: bad argument");
+    if (count == 0) return MG_OK;
+    MG_REQUIRE(keys && workspace && order && sorted_keys, "mg_sort_by_key: null pointer");
+    hipStream_t st = (hipStream_t)stream;
+    const int chunks = (int)ceil_div(count, kSortChunk);
+    int* counts = static_cast<int*>(workspace);
+    int* totals = counts + (long)chunks * kDigits;
+    int *spare_keys = totals + kDigits, *spare_values = spare_keys + count;
+    int passes = 1;
+    while (passes < 4 && ((long)key_limit - 1) >> (kDigitBits * passes)) passes++;
+    const int *k_in = keys, *v_in = nullptr;
+    for (int p = 0; p < passes; p++) {
+        // the last pass ends in the caller's arrays
+        const bool to_out = (passes - 1 - p) % 2 == 0;
+        int *k_out = to_out ? sorted_keys : spare_keys, *v_out = to_out ? order : spare_values;
+        hipLaunchKernelGGL(sort_count_kernel, dim3(chunks), dim3(256), 0, st, k_in, count, kDigitBits * p, chunks, counts);
+        hipLaunchKernelGGL(sort_prefix_kernel, dim3(kDigits), dim3(64), 0, st, counts, chunks, totals);
+        hipLaunchKernelGGL(sort_scatter_kernel, dim3(chunks), dim3(256), 0, st, k_in, v_in, count, kDigitBits * p, chunks, counts,
+                           totals, k_out, v_out);
+        k_in = k_out;
+        v_in = v_out;
+    }
+    return check_launch("mg_sort_by_key");
+}
+
+}  // extern "C"

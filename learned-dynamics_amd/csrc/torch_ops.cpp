@@ -989,6 +989,64 @@ std::tuple<std::vector<OptTensor>, Tensors> painn_update_train_bwd(const at::Ten
     return {g_x, params};
 }
 
+// (order, sorted keys) of a stable sort of int32 keys in 0 .. limit - 1
+std::pair<at::Tensor, at::Tensor> sort_by_key(const at::Tensor& keys, int64_t limit) {
+    check_input(keys, "keys", at::kInt);
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(keys.device());
+    at::Tensor order = at::empty_like(keys), sorted = at::empty_like(keys);
+    size_t n = 0;
+    check(mg_sort_by_key_workspace_bytes(keys.numel(), &n));
+    at::Tensor ws = bytes_like(keys, n);
+    check(mg_sort_by_key(keys.data_ptr<int>(), keys.numel(), (int)limit, ws.data_ptr(), order.data_ptr<int>(), sorted.data_ptr<int>(),
+                         stream_of(keys)));
+    return {order, sorted};
+}
+
+// (d_table, d_actv, d_v) of the message interpolated from its grid; each only if wanted
+std::tuple<OptTensor, OptTensor, OptTensor> painn_grid_message_bwd(const at::Tensor& table, const at::Tensor& actv,
+                                                                   const at::Tensor& actv_sliced, const at::Tensor& v,
+                                                                   const at::Tensor& r_ij, const at::Tensor& g_v, const at::Tensor& g_a,
+                                                                   const at::Tensor& src, const at::Tensor& dst,
+                                                                   const at::Tensor& row_ptr, const OptTensor& order,
+                                                                   const OptTensor& node_order, double period, double epsilon,
+                                                                   bool want_table, bool want_actv, bool want_v) {
+    for (const at::Tensor& t : {table, actv, actv_sliced, v, r_ij, g_v, g_a}) check_input(t, "operand of the message");
+    for (const at::Tensor& t : {src, dst, row_ptr}) check_input(t, "index", at::kInt);
+    for (const OptTensor& t : {order, node_order})
+        if (t.has_value()) check_input(*t, "order", at::kInt);
+    const int64_t N = v.size(0), n = v.size(1), E = r_ij.size(0), rows = table.size(0);
+    TORCH_CHECK(actv.numel() == N * 4 * n && actv_sliced.numel() == N * 4 * n && v.numel() == N * n * 3 && table.size(1) == 4 * n &&
+                    g_v.numel() == N * n * 3 && g_a.numel() == N * n && r_ij.numel() == 3 * E && src.numel() == E && dst.numel() == E &&
+                    row_ptr.numel() == N + 1 && (!order.has_value() || order->numel() == E) &&
+                    (!node_order.has_value() || node_order->numel() == N),
+                "painn_grid_message_bwd: operand sizes");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(v.device());
+    const mg_stream_t st = stream_of(v);
+    size_t n_ws = 0;
+    check(mg_painn_grid_grad_workspace_bytes((int)rows, (int)n, E, &n_ws));
+    at::Tensor ws = bytes_like(v, n_ws);
+    auto ints = [](const OptTensor& t) { return t.has_value() ? t->data_ptr<int>() : nullptr; };
+    OptTensor d_table, d_actv, d_v;
+    if (want_actv || want_v) {
+        if (want_actv) d_actv = floats(v, {N, 4 * n});
+        if (want_v) d_v = floats(v, v.sizes());
+        check(mg_painn_grid_node_grad(row_ptr.data_ptr<int>(), ints(order), src.data_ptr<int>(), ints(node_order), (int)N, E, fp(r_ij),
+                                      fp(table), (int)rows, (float)period, (float)epsilon, fp(g_v), fp(g_a), fp(actv), fp(v), (int)n,
+                                      ws.data_ptr(), want_actv ? fp(*d_actv) : nullptr, want_v ? fp(*d_v) : nullptr, st));
+    }
+    if (want_table) {
+        d_table = floats(v, table.sizes());
+        at::Tensor key = at::empty({E}, src.options()), ptr = at::empty({rows + 1}, src.options());
+        check(mg_painn_grid_rows(fp(r_ij), E, (int)rows, (float)period, key.data_ptr<int>(), st));
+        auto [by_row, sorted] = sort_by_key(key, rows);
+        check(mg_segment_row_ptr(sorted.data_ptr<int>(), 0, E, (int)rows, ptr.data_ptr<int>(), st));
+        check(mg_painn_grid_table_grad(by_row.data_ptr<int>(), ptr.data_ptr<int>(), src.data_ptr<int>(), dst.data_ptr<int>(), (int)N, E,
+                                       fp(r_ij), (int)rows, (float)period, (float)epsilon, fp(g_v), fp(g_a), fp(actv_sliced), fp(v),
+                                       (int)n, ws.data_ptr(), fp(*d_table), st));
+    }
+    return {d_table, d_actv, d_v};
+}
+
 }  // namespace
 
 void register_ops(pybind11::module_& m) {
@@ -1005,6 +1063,8 @@ void register_ops(pybind11::module_& m) {
     m.def("painn_update", &painn_update);
     m.def("painn_message_grid", &painn_message_grid);
     m.def("painn_message_edges", &painn_message_edges);
+    m.def("sort_by_key", &sort_by_key);
+    m.def("painn_grid_message_bwd", &painn_grid_message_bwd);
     m.def("mlp_silu_fwd", &mlp_silu_fwd);
     m.def("mlp_silu_bwd", &mlp_silu_bwd);
     m.def("edge_encode_fwd", &edge_encode_fwd);

@@ -715,9 +715,11 @@ class _PainnGridMessage(torch.autograd.Function):
     """(grid (rows, 4n), actv (nodes, 4n), v (nodes, n, 3)) -> (out_v, out_a) of the message for edge vectors that are
     not differentiated, with the filter interpolated from the grid.  Forward: the inference kernel of the layer
     (mg_painn_table_message: lengths, directions, interpolation, the lines 94-100 of archs/meanflow_painn8.py and the
-    sum over the edges of a node in one pass; no per-edge filter is stored).  Backward: the gradient kernel of the
-    unfused formulation with the filter of every edge interpolated again inside it and the gradients of actv and v
-    summed per destination inside it (mg_painn_combine_bwd_rows), then the scatter into the grid.  A recorded backward pass differentiates the unfused formulation instead."""
+    sum over the edges of a node in one pass; no per-edge filter is stored).  Backward: where the grid fits in LDS, one
+    kernel for the gradients of actv and v and one, over the edges sorted by grid row, for the grid's
+    (mg_painn_grid_node_grad, mg_painn_grid_table_grad: nothing per edge is stored); for larger grids the gradient kernel of
+    the unfused formulation with the filter of every edge interpolated again inside it (mg_painn_combine_bwd_rows), then
+    the scatter into the grid.  A recorded backward pass differentiates the unfused formulation instead."""
 
     @staticmethod
     def forward(ctx, table, actv, v, r_ij, graph, period, epsilon):
@@ -728,6 +730,7 @@ class _PainnGridMessage(torch.autograd.Function):
         if table.size(0) <= ops.PAINN_SLICED_MAX_ROWS and n % ops.PAINN_SLICE == 0:
             # the grid fits in LDS: the kernel that holds it there takes actv with its columns grouped slice by slice
             actv_s = actv[:, _slice_permutation(n, actv.device)].contiguous()
+            ctx.actv_s = actv_s if ctx.needs_input_grad[0] else None
             out_a, out_v = ops.painn_table_message_sliced(graph.row_ptr, graph.dst32, r_ij, table, period, actv_s, v, epsilon,
                                                           node_order=getattr(graph, "cell_order", None))
         else:
@@ -745,6 +748,12 @@ class _PainnGridMessage(torch.autograd.Function):
                 grads = torch.autograd.grad(out, leaves, (g_v, g_a), create_graph=True, allow_unused=True)
             return tuple(g if nd else None for g, nd in zip(grads, need)) + (None, None, None, None)
         by_dst, by_src = graph.by_dst, graph.by_src
+        if ops.painn_grid_grad_supported(table.size(0), v.size(1)) and all(t.data_ptr() % 16 == 0 for t in (table, v, actv)):
+            actv_s = ctx.actv_s if need[0] else actv              # (read for the grid's gradient only)
+            grads = ops.painn_grid_message_bwd(table, actv, actv_s, v, r_ij, g_v.contiguous(), g_a.contiguous(), graph.src32,
+                                               graph.dst32, by_dst.row_ptr, by_dst.perm, getattr(graph, "cell_order", None),
+                                               ctx.period, ctx.epsilon, need[0], need[1], need[2])
+            return (*grads, None, None, None, None)
         d = torch.linalg.vector_norm(r_ij, dim=-1).contiguous()
         want = (bool(need[0]), bool(need[1]), bool(need[2]), False)
         # (actv and v are read at an edge's destination: their gradients are summed over a destination's edges inside)

@@ -103,15 +103,18 @@ class _SortedIndex:
         if self._perm is None:
             # stable sort by destination: index plumbing, done once per graph and only when a
             # gradient through a gather-by-dst is asked for
-            self._perm = torch.sort(self.index.long(), stable=True).indices.to(torch.int32).contiguous()
+            self._perm, ordered = ops.sort_by_key(self.index, self.n_rows)
+            if self._row_ptr is None:
+                self._row_ptr = ops.segment_row_ptr(ordered, self.n_rows)
         return self._perm
 
     @property
     def row_ptr(self):
         if self._row_ptr is None:
-            # integer gather (a float32 detour would round node ids above 2^24)
-            idx = self.index if self.is_sorted else self.index[self.perm.long()]
-            self._row_ptr = ops.segment_row_ptr(idx.contiguous(), self.n_rows)
+            if self.is_sorted:
+                self._row_ptr = ops.segment_row_ptr(self.index.contiguous(), self.n_rows)
+            else:
+                self.perm                                # (leaves the row pointer behind)
         return self._row_ptr
 
 

@@ -377,6 +377,11 @@ def edge_vectors(pos, src, dst, box, want_shift=False):
 
 
 # --------------------------------------------------------------------- stage C
+def sort_by_key(keys, limit):
+    """(order, sorted keys), int32: a stable sort of int32 keys in 0 .. limit - 1."""
+    return _ext.sort_by_key(keys, max(int(limit), 1))
+
+
 def segment_row_ptr(index, n_rows):
     if index.dtype not in (torch.int32, torch.int64):
         raise RuntimeError("index must be int32 or int64")
@@ -1187,6 +1192,7 @@ mlp_silu_bwd = _ext.mlp_silu_bwd
 painn_edge_encode_fwd = _ext.edge_encode_fwd
 painn_edge_encode_bwd = _ext.edge_encode_bwd
 painn_combine_dual_bwd = _ext.combine_dual_bwd
+painn_grid_message_bwd = _ext.painn_grid_message_bwd
 painn_update_train_fwd = _ext.painn_update_train_fwd
 painn_update_train_bwd = _ext.painn_update_train_bwd
 
@@ -1591,6 +1597,10 @@ def painn_combine_bwd_rows(dist, actv, v, direction, dm, da, row_ptr, order, gra
     return d_dist, d_actv, dv, d_dir
 
 
+def painn_grid_grad_supported(table_rows, n):
+    return bool(_lib.mg_painn_grid_grad_supported(int(table_rows), int(n)))
+
+
 def painn_table_interp_supported(table_rows, cols):
     return bool(_lib.mg_painn_table_interp_supported(int(table_rows), int(cols)))
 
@@ -1622,8 +1632,8 @@ def painn_table_sorted_edges(d, table_rows, period):
     with _on(d.device):
         bucket = torch.empty(E, dtype=torch.int32, device=d.device)
         L.check(_lib.mg_painn_table_buckets(_p(d), E, int(table_rows), float(period), _p(bucket), _stream()))
-        ordered, perm = torch.sort(bucket, stable=True)
-    return perm.to(torch.int32).contiguous(), segment_row_ptr(ordered.contiguous(), int(table_rows))
+    perm, ordered = sort_by_key(bucket, int(table_rows))
+    return perm, segment_row_ptr(ordered, int(table_rows))
 
 
 def painn_table_interp_bwd(g, table, d, period, perm, bucket_ptr, want_length_grad=True, order=0, table_rows=None):

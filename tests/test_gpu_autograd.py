@@ -961,3 +961,39 @@ def test_painn_layers_of_values_and_tangents(pkg, B, N, n, n_rbf, degree):
     g_o = torch.autograd.grad(total(f_o(*x_o), lambda w: w.double()), x_o + params_o)
     for k, (a, b) in enumerate(zip(g_d, g_o)):
         _close(a, b, f"gradient {k}", 1.6e-5)
+
+
+@pytest.mark.parametrize("n,rows,N,E,seed", [(16, 4, 3, 40, 0), (32, 64, 50, 3000, 1), (128, 512, 700, 20000, 2), (256, 512, 33, 5, 3),
+                                            (128, 512, 40, 500000, 4)])
+def test_gradients_of_the_message_from_its_grid(pkg, ops, n, rows, N, E, seed):
+    """painn_grid_message_bwd against the unfused formulation differentiated in float64: grids from 4 rows to what LDS holds, one
+    slice of channels and sixteen, fewer edges than a step of a wave, rows without edges, several pieces per grid row.
+    Tolerance: a gradient is a sum of at most E products rounded to 2^-24 each, 8 2^-24 sqrt(E) of the largest entry, and the
+    fraction of an edge between grid rows carries rows 2^-24."""
+    g = torch.Generator().manual_seed(0x947 + seed)
+    period, eps = 10.0, 0.1
+    src = torch.sort(torch.randint(0, N, (E,), generator=g)).values
+    dst = torch.randint(0, max(1, N - 1), (E,), generator=g)
+    u = torch.randn(E, 3, generator=g)
+    r = (u / u.norm(dim=-1, keepdim=True) * (0.05 + 4.9 * torch.rand(E, 1, generator=g)))
+    k = torch.arange(rows)[:, None] / rows * 2 * torch.pi
+    table = torch.randn(1, 4 * n, generator=g) * torch.cos(k + torch.randn(1, 4 * n, generator=g))      # smooth along the grid
+    actv, v = torch.randn(N, 4 * n, generator=g), torch.randn(N, n, 3, generator=g)
+    g_v, g_a = torch.randn(N, n, 3, generator=g), torch.randn(N, n, generator=g)
+    gl = importlib.import_module("learned-dynamics_amd.graph_layers")
+    graph = gl.Graph(src.cuda(), dst.cuda(), None, 1, N)
+    order, ordered = ops.sort_by_key(graph.dst32, N)
+    assert torch.equal(order.cpu().long(), torch.sort(dst, stable=True).indices) and torch.equal(ordered.cpu().long(), torch.sort(dst).values)
+    T, A, V = (t.double().requires_grad_() for t in (table, actv, v))
+    rd = r.double()
+    diff = importlib.import_module("learned-dynamics_amd.differentiable")
+    f = diff._table_interp_plain(T, rd.norm(dim=-1), period)
+    m, a = diff._painn_combine_plain(f, A[dst], V[dst], rd / torch.sqrt(eps + (rd ** 2).sum(-1, keepdim=True)))
+    ref = torch.autograd.grad((m * g_v.double()[src]).sum() + (a * g_a.double()[src]).sum(), (T, A, V))
+    perm = ops.painn_slice_permutation(n, "cuda")
+    got = ops.painn_grid_message_bwd(table.cuda(), actv.cuda(), actv.cuda()[:, perm].contiguous(), v.cuda(), r.cuda(), g_v.cuda(),
+                                     g_a.cuda(), graph.src32, graph.dst32, graph.by_dst.row_ptr, graph.by_dst.perm, None, period,
+                                     eps, True, True, True)
+    for name, x, y in zip(("grid", "actv", "v"), got, ref):
+        err = float((x.cpu().double() - y).abs().max() / y.abs().max())
+        assert err <= 2 ** -24 * (8 * E ** 0.5 + rows), f"{name}: {err:.3g}"
