@@ -597,7 +597,7 @@ int mg_sort_by_key(const int* keys, long count, int key_limit, void* workspace, 
  * 16-byte aligned.  *_rowmax: upper bounds of the row maxima of what was written, which the linears scale by.
  *
  * The activation of a layer: h = SiLU(z), h_t = SiLU'(z) z_t, and its adjoint. */
-int mg_silu_rows_fwd(const float* z, long rows, int n, int dual, float* h, mg_stream_t stream);
+int mg_silu_rows_fwd(const float* z, long rows, int n, int dual, float* h, float* h_rowmax, mg_stream_t stream);
 int mg_silu_rows_bwd(const float* z, const float* dh, long rows, int n, int dual, float* dz, float* dz_rowmax, mg_stream_t stream);
 /* Edge vectors r (E, 3) [and tangents r_t] -> enc = radial_encode(r, n, rmax) ((1 or 2) E, n) and dir = r / sqrt(|r|^2 + eps)
  * [and dir_t]; the adjoint gives g_r [and g_r_t].  r_t == NULL: values alone. */

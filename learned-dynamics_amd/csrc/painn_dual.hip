@@ -86,21 +86,40 @@ __device__ __forceinline__ float max4(float m, const F4& v) {
 }
 
 // ------------------------------------------------------------------------------------------------ activation of a layer
-// h = SiLU(z), h_t = SiLU'(z) z_t
+// h = SiLU(z), h_t = SiLU'(z) z_t, and the row maxima of both
 template <bool DUAL>
-__global__ void __launch_bounds__(256) silu_rows_fwd_kernel(const float* __restrict__ z, long count, float* __restrict__ h) {
-    for (long k = 4 * ((long)blockIdx.x * 256 + threadIdx.x); k < count; k += 1024L * gridDim.x) {
+__global__ void __launch_bounds__(256) silu_rows_fwd_kernel(const float* __restrict__ z, long R, int n, int lanes,
+                                                            float* __restrict__ h, float* __restrict__ h_max) {
+    const long t = (long)blockIdx.x * 256 + threadIdx.x;
+    const long r_raw = t / lanes;
+    const bool live = r_raw < R;
+    const long r = live ? r_raw : R - 1;
+    const int lane = (int)(t - r_raw * lanes);
+    const long half = R * n;
+    float mx = 0.f, mxt = 0.f;
+    for (int c = 4 * lane; c < n; c += 4 * lanes) {
+        const long k = r * n + c;
         const F4 v = ld4(z + k);
-        F4 t, r, rt;
-        if constexpr (DUAL) t = ld4(z + count + k);
+        F4 vt, o, ot;
+        if constexpr (DUAL) vt = ld4(z + half + k);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const Silu s = silu(v.f[j]);
-            r.f[j] = s.f;
-            if constexpr (DUAL) rt.f[j] = s.d1 * t.f[j];
+            o.f[j] = s.f;
+            if constexpr (DUAL) ot.f[j] = s.d1 * vt.f[j];
         }
-        st4(h + k, r);
-        if constexpr (DUAL) st4(h + count + k, rt);
+        mx = max4(mx, o);
+        if (live) st4(h + k, o);
+        if constexpr (DUAL) {
+            mxt = max4(mxt, ot);
+            if (live) st4(h + half + k, ot);
+        }
+    }
+    mx = group_max(mx, lanes);
+    if constexpr (DUAL) mxt = group_max(mxt, lanes);
+    if (live && lane == 0) {
+        h_max[r] = mx;
+        if constexpr (DUAL) h_max[R + r] = mxt;
     }
 }
 
@@ -874,12 +893,12 @@ using namespace mg;
 
 extern "C" {
 
-int mg_silu_rows_fwd(const float* z, long rows, int n, int dual, float* h, mg_stream_t stream) {
-    MG_REQUIRE(rows_ok(rows, n) && z && h && aligned16(z) && aligned16(h), "mg_silu_rows_fwd: n % 4 == 0 and aligned arrays expected");
+int mg_silu_rows_fwd(const float* z, long rows, int n, int dual, float* h, float* h_rowmax, mg_stream_t stream) {
+    MG_REQUIRE(rows_ok(rows, n) && z && h && h_rowmax && aligned16(z) && aligned16(h),
+               "mg_silu_rows_fwd: n % 4 == 0 and aligned arrays expected");
     if (rows == 0) return MG_OK;
-    const long blocks = ceil_div(rows * n / 4, 256);
-    const dim3 grid((unsigned)(blocks < 4096 ? blocks : 4096)), block(256);
-    MG_DUAL_LAUNCH(silu_rows_fwd_kernel, grid, block, z, rows * n, h);
+    const int lanes = row_lanes(n);
+    MG_DUAL_LAUNCH(silu_rows_fwd_kernel, dim3(row_blocks(rows, lanes)), dim3(256), z, rows, n, lanes, h, h_rowmax);
     return check_launch("mg_silu_rows_fwd");
 }
 

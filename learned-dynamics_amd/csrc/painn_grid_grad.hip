@@ -20,6 +20,7 @@ __device__ __forceinline__ void st4(float* p, float4 v) { *reinterpret_cast<floa
 
 // |r| / h and 1 / sqrt(eps + |r|^2).  (The fused multiply-adds are spelled out: every kernel here that puts an edge into a grid
 // row must find the same one.)
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 struct EdgePlace { float u, inv; };
 __device__ __forceinline__ EdgePlace place(float x, float y, float z, float inv_h, float eps) {
     const float r2 = fmaf(x, x, fmaf(y, y, z * z));
@@ -178,15 +179,17 @@ __global__ void __launch_bounds__(256) grid_row_grad_kernel(const int* __restric
     const float* v_base = v + (slice * kSliceChan + 4 * l4) * 3;
     const float* gv_base = g_v + (slice * kSliceChan + 4 * l4) * 3;
     const float* ga_base = g_a + slice * kSliceChan + 4 * l4;
-    float acc[4][16];                                         // tap j; value 4 k + c
+    // value 4 k + c of the four taps.  Each is a sum of outer products of an edge's 4 weights with its 4 lanes' values: the
+    // 16-block 4 x 4 x 1 matrix instruction in fp32 (block = edge slot, row = tap, column = lane of the slot)
+    floatx4 acc[16];
 #pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int k = 0; k < 16; k++) acc[j][k] = 0.f;
+    for (int k = 0; k < 16; k++) acc[k] = floatx4{0.f, 0.f, 0.f, 0.f};
     long e = lo + 16 * wave + sub;
     float4 ra = make_float4(0.f, 0.f, 0.f, 0.f), rb = ra;
     if (e < hi) { ra = rec[2 * e]; rb = rec[2 * e + 1]; }
-    while (e < hi) {
+    // (a slot past the end takes part in the matrix instructions with weight zero)
+    for (long e0 = lo + 16 * wave; e0 < hi; e0 += 64) {
+        const bool live = e < hi;
         const long from = min(max((long)__float_as_int(ra.x), 0L), n_nodes - 1), to = min(max((long)__float_as_int(ra.y), 0L), n_nodes - 1);
         const float* ap = a_base + to * 4 * n;
         const float* vp = v_base + to * 3 * n;
@@ -202,6 +205,7 @@ __global__ void __launch_bounds__(256) grid_row_grad_kernel(const int* __restric
         const float ux = ra.w, uy = rb.x, uz = rb.y;
         float w[4];
         lagrange(ra.z, w);
+        const float my_w = live ? (l4 == 0 ? w[0] : l4 == 1 ? w[1] : l4 == 2 ? w[2] : w[3]) : 0.f;
         const float vv[12] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w, v2.x, v2.y, v2.z, v2.w};
         const float gg[12] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w, g2.x, g2.y, g2.z, g2.w};
         const float gs[4] = {ga.x, ga.y, ga.z, ga.w};
@@ -217,14 +221,17 @@ __global__ void __launch_bounds__(256) grid_row_grad_kernel(const int* __restric
                                 ((uy * z - uz * y) * vx + (uz * x - ux * z) * vy + (ux * y - uy * x) * vz) * av[1],
                                 (ux * x + uy * y + uz * z) * av[2], gs[c] * av[3]};
 #pragma unroll
-            for (int k = 0; k < 4; k++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[j][4 * k + c] = fmaf(w[j], d[k], acc[j][4 * k + c]);
+            for (int k = 0; k < 4; k++) acc[4 * k + c] = __builtin_amdgcn_mfma_f32_4x4x1f32(my_w, d[k], acc[4 * k + c], 0, 0, 0);
         }
         ra = na; rb = nb;
     }
 #pragma unroll
-    for (int j = 0; j < 4; j++) fold[wave][j][lane] = sum_over_slots(acc[j], lane);
+    for (int j = 0; j < 4; j++) {
+        float tap[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) tap[k] = acc[k][j];
+        fold[wave][j][lane] = sum_over_slots(tap, lane);
+    }
     __syncthreads();
     // wave j adds tap j over the four waves; value `sub` = 4 k + c of the channel quad l4
     const float sum = (fold[0][wave][lane] + fold[1][wave][lane]) + (fold[2][wave][lane] + fold[3][wave][lane]);

@@ -293,16 +293,27 @@ __global__ void __launch_bounds__(256) absmax_parts_kernel(const float* __restri
     __syncthreads();
     if (threadIdx.x == 0) parts[blockIdx.x] = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
 }
-// the same for an array of any length and alignment (bounds handed in by the caller)
-__global__ void __launch_bounds__(256) absmax_parts_scalar_kernel(const float* __restrict__ x, long n,
-                                                                  float* __restrict__ parts) {
+// the same for one or two arrays of any length and alignment (bounds handed in by the caller) in one launch: the first
+// blocks_a workgroups take the first array
+struct BoundArray {
+    const float* data;
+    long n;
+    float* parts;
+    int blocks;
+};
+__global__ void __launch_bounds__(256) absmax_parts_scalar_kernel(const BoundArray a, const BoundArray b) {
+    const bool first = (int)blockIdx.x < a.blocks;
+    const float* __restrict__ x = first ? a.data : b.data;
+    const long n = first ? a.n : b.n, stride = 256L * (first ? a.blocks : b.blocks);
+    const int block = first ? blockIdx.x : blockIdx.x - a.blocks;
+    float* __restrict__ parts = first ? a.parts : b.parts;
     float m = 0.f;
-    for (long k = (long)blockIdx.x * 256 + threadIdx.x; k < n; k += (long)gridDim.x * 256) m = fmaxf(m, fabsf(x[k]));
+    for (long k = (long)block * 256 + threadIdx.x; k < n; k += stride) m = fmaxf(m, fabsf(x[k]));
     for (int d = 1; d < 64; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
     __shared__ float wave_max[4];
     if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0) parts[blockIdx.x] = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
+    if (threadIdx.x == 0) parts[block] = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
 }
 
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) wgrad_f16x2_kernel(const float* __restrict__ dy, const float* __restrict__ x,
@@ -611,20 +622,21 @@ int mg_tensor_linear_wgrad_f16x2_rows(const float* dy, const float* x, const flo
     float* maxima = part + splits * n;                       // [dy: kFParts][x: kFParts]
     float* colsum_part = db ? maxima + 2 * kFParts : nullptr; // [slice][dim_out]
     constexpr long kDirectBounds = 16384;                    // a bound array this short is read by every workgroup itself
-    auto bound_parts = [&](const float* data, long count, const float* bound, long n_bound, float* parts) -> int {
-        // partial maxima of the caller's bounds, or of the data itself
+    auto blocks_for = [](long len) { return (int)(ceil_div(len, 4096) < kFParts ? ceil_div(len, 4096) : kFParts); };
+    BoundArray scan[2] = {};
+    // partial maxima of the caller's bounds, or of the data itself
+    auto bound_parts = [&](BoundArray& a, const float* data, long count, const float* bound, long n_bound, float* parts) -> int {
         if (bound && n_bound <= kDirectBounds) return (int)n_bound;
-        const float* from = bound ? bound : data;
-        const long len = bound ? n_bound : count;
-        const int blocks = (int)(ceil_div(len, 4096) < kFParts ? ceil_div(len, 4096) : kFParts);
-        if (bound)
-            hipLaunchKernelGGL(absmax_parts_scalar_kernel, dim3(blocks), dim3(256), 0, st, from, len, parts);
-        else
-            hipLaunchKernelGGL(absmax_parts_kernel, dim3(blocks), dim3(256), 0, st, from, len, parts);
+        const int blocks = blocks_for(bound ? n_bound : count);
+        if (bound) a = BoundArray{bound, n_bound, parts, blocks};
+        else hipLaunchKernelGGL(absmax_parts_kernel, dim3(blocks), dim3(256), 0, st, data, count, parts);
         return blocks;
     };
-    const int na = bound_parts(dy, rows * dim_out, dy_bound, n_dy_bound, maxima);
-    const int nb = bound_parts(x, rows * dim_in, x_bound, n_x_bound, maxima + kFParts);
+    const int na = bound_parts(scan[0], dy, rows * dim_out, dy_bound, n_dy_bound, maxima);
+    const int nb = bound_parts(scan[1], x, rows * dim_in, x_bound, n_x_bound, maxima + kFParts);
+    if (scan[0].blocks + scan[1].blocks > 0)
+        hipLaunchKernelGGL(absmax_parts_scalar_kernel, dim3((unsigned)(scan[0].blocks + scan[1].blocks)), dim3(256), 0, st, scan[0],
+                           scan[1]);
     const float* dy_parts = (dy_bound && n_dy_bound <= kDirectBounds) ? dy_bound : maxima;
     const float* x_parts = (x_bound && n_x_bound <= kDirectBounds) ? x_bound : maxima + kFParts;
     dim3 grid((unsigned)ceil_div(dim_out, kFTile), (unsigned)ceil_div(dim_in, kFTile), (unsigned)splits), block(256);

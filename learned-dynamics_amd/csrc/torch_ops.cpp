@@ -669,18 +669,14 @@ void pack_ahead(const Tensors& weights) {
     }
 }
 
-// y = x W^T, with the bias added to the first bias_rows rows; ymax: row bounds of y where the kernel that runs emits them
-at::Tensor rows_linear(const at::Tensor& W, const OptTensor& bias, const at::Tensor& x, int64_t bias_rows, Bound bound,
-                       OptTensor* ymax = nullptr) {
+// y = x W^T, with the bias added to the first bias_rows rows
+at::Tensor rows_linear(const at::Tensor& W, const OptTensor& bias, const at::Tensor& x, int64_t bias_rows, Bound bound) {
     const int64_t rows = x.size(0), dim_in = W.size(1), dim_out = W.size(0);
     at::Tensor y = floats(x, {rows, dim_out});
     if (rows == 0) return y;
     if (mg_get_linear_mode() == kModeF16x2 && f16x2_takes(rows, dim_in, dim_out, x)) {
         if (!bound.base.has_value()) bound = Bound{row_absmax(x)};
-        at::Tensor m;
-        if (ymax) m = floats(x, {rows, rowmax_parts(rows, dim_in, dim_out, false)});
-        run_f16x2(W, dim_in, fp(x), rows, bound, bias, kActNone, false, 1, y, ymax ? &m : nullptr, false, bias_rows);
-        if (ymax) *ymax = m;
+        run_f16x2(W, dim_in, fp(x), rows, bound, bias, kActNone, false, 1, y, nullptr, false, bias_rows);
         return y;
     }
     auto piece = [&](int64_t lo, int64_t hi, const OptTensor& b) {
@@ -714,9 +710,6 @@ std::pair<at::Tensor, OptTensor> rows_wgrad(const at::Tensor& dy, const at::Tens
     return {dW, want_bias ? OptTensor(dy.narrow(0, 0, bias_rows).sum(0)) : OptTensor()};
 }
 
-// |SiLU(z)| <= |z| and |SiLU'(z)| <= 1.0999
-constexpr float kSiluSlope = 1.1f;
-
 // Linear, SiLU, Linear, SiLU, Linear on S = [x; x_t] (R or 2 R rows): y and what the adjoint reads again
 std::pair<at::Tensor, std::vector<OptTensor>> mlp_rows_fwd(const at::Tensor& S, int64_t R, OptTensor bound, const Tensors& W,
                                                            const Tensors& b, bool train) {
@@ -728,12 +721,11 @@ std::pair<at::Tensor, std::vector<OptTensor>> mlp_rows_fwd(const at::Tensor& S, 
     at::Tensor h = S;
     Bound hb{bound};
     for (int l = 0; l < 2; l++) {
-        OptTensor m;
-        at::Tensor z = rows_linear(W[l], OptTensor(b[l]), h, R, hb, &m);
+        at::Tensor z = rows_linear(W[l], OptTensor(b[l]), h, R, hb), m = floats(z, {z.size(0), 1});
         h = floats(z, z.sizes());
-        check(mg_silu_rows_fwd(fp(z), R, (int)z.size(1), dual, fp(h), stream_of(z)));
-        hb = Bound{m, dual ? kSiluSlope : 1.f};
-        saved.insert(saved.end(), {OptTensor(z), m, OptTensor(h)});
+        check(mg_silu_rows_fwd(fp(z), R, (int)z.size(1), dual, fp(h), fp(m), stream_of(z)));
+        hb = Bound{OptTensor(m)};
+        saved.insert(saved.end(), {OptTensor(z), OptTensor(m), OptTensor(h)});
     }
     return {rows_linear(W[2], OptTensor(b[2]), h, R, hb), saved};
 }
