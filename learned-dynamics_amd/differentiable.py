@@ -218,16 +218,16 @@ class _MlpSilu(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, x_t, bound, *params):
-        ctx.save_for_backward(x, x_t, *params)
         train = any(ctx.needs_input_grad)
-        y, y_t, saved = ops.mlp_silu_fwd(x, x_t, bound, params[0::2], params[1::2], train)
-        ctx.rows_saved = saved if train else None
+        y, y_t, rows = ops.mlp_silu_fwd(x, x_t, bound, params[0::2], params[1::2], train)
+        ctx.save_for_backward(x, x_t, *params, *(rows if train else ()))
         ctx.set_materialize_grads(False)
         return y if x_t is None else (y, y_t)
 
     @staticmethod
     def backward(ctx, g, g_t=None):
-        x, x_t, *params = ctx.saved_tensors
+        x, x_t, *saved = ctx.saved_tensors
+        params, rows = saved[:6], saved[6:]
         need = list(ctx.needs_input_grad)
         if g is None and g_t is None:
             return (None,) * len(need)
@@ -240,7 +240,7 @@ class _MlpSilu(torch.autograd.Function):
             g, need[8] = torch.zeros_like(g_t), False                       # the last bias
         if x_t is not None and g_t is None:
             g_t, need[1] = torch.zeros_like(g), False
-        g_x, g_xt, d_params = ops.mlp_silu_bwd(g.contiguous(), _dense(g_t), x, x_t, params[0::2], ctx.rows_saved,
+        g_x, g_xt, d_params = ops.mlp_silu_bwd(g.contiguous(), _dense(g_t), x, x_t, params[0::2], rows,
                                                need[0] or need[1], any(need[3:]))
         return (g_x if need[0] else None, g_xt if need[1] else None, None) \
             + tuple(d if nd else None for d, nd in zip(d_params, need[3:]))
@@ -725,21 +725,21 @@ class _PainnGridMessage(torch.autograd.Function):
     def forward(ctx, table, actv, v, r_ij, graph, period, epsilon):
         ctx.graph, ctx.period, ctx.epsilon = graph, period, epsilon
         table, actv, v = table.contiguous(), actv.contiguous(), v.contiguous()
-        ctx.save_for_backward(table, actv, v, r_ij)
+        actv_s = None
         n = v.size(1)
         if table.size(0) <= ops.PAINN_SLICED_MAX_ROWS and n % ops.PAINN_SLICE == 0:
             # the grid fits in LDS: the kernel that holds it there takes actv with its columns grouped slice by slice
             actv_s = actv[:, _slice_permutation(n, actv.device)].contiguous()
-            ctx.actv_s = actv_s if ctx.needs_input_grad[0] else None
             out_a, out_v = ops.painn_table_message_sliced(graph.row_ptr, graph.dst32, r_ij, table, period, actv_s, v, epsilon,
                                                           node_order=getattr(graph, "cell_order", None))
         else:
             out_a, out_v = ops.painn_table_message(graph.row_ptr, graph.dst32, r_ij, table, period, actv, v, epsilon)
+        ctx.save_for_backward(table, actv, v, r_ij, actv_s if ctx.needs_input_grad[0] else None)
         return out_v, out_a
 
     @staticmethod
     def backward(ctx, g_v, g_a):
-        table, actv, v, r_ij = ctx.saved_tensors
+        table, actv, v, r_ij, actv_s = ctx.saved_tensors
         graph, need = ctx.graph, ctx.needs_input_grad
         if torch.is_grad_enabled():
             with torch.enable_grad():
@@ -749,10 +749,11 @@ class _PainnGridMessage(torch.autograd.Function):
             return tuple(g if nd else None for g, nd in zip(grads, need)) + (None, None, None, None)
         by_dst, by_src = graph.by_dst, graph.by_src
         if ops.painn_grid_grad_supported(table.size(0), v.size(1)) and all(t.data_ptr() % 16 == 0 for t in (table, v, actv)):
-            actv_s = ctx.actv_s if need[0] else actv              # (read for the grid's gradient only)
-            grads = ops.painn_grid_message_bwd(table, actv, actv_s, v, r_ij, g_v.contiguous(), g_a.contiguous(), graph.src32,
-                                               graph.dst32, by_dst.row_ptr, by_dst.perm, getattr(graph, "cell_order", None),
-                                               ctx.period, ctx.epsilon, need[0], need[1], need[2])
+            # (the sliced rows are read for the grid's gradient only)
+            grads = ops.painn_grid_message_bwd(table, actv, actv if actv_s is None else actv_s, v, r_ij, g_v.contiguous(),
+                                               g_a.contiguous(), graph.src32, graph.dst32, by_dst.row_ptr, by_dst.perm,
+                                               getattr(graph, "cell_order", None), ctx.period, ctx.epsilon, need[0], need[1],
+                                               need[2])
             return (*grads, None, None, None, None)
         d = torch.linalg.vector_norm(r_ij, dim=-1).contiguous()
         want = (bool(need[0]), bool(need[1]), bool(need[2]), False)
@@ -809,17 +810,17 @@ class _PainnUpdate(torch.autograd.Function):
     @staticmethod
     def forward(ctx, upd, x_a, x_at, x_v, x_vt, *params):
         ctx.upd = upd
-        ctx.save_for_backward(x_a, x_at, x_v, x_vt, *params)
-        outs, saved = ops.painn_update_train_fwd(x_a, x_at, x_v, x_vt, params[:3], params[5::2], params[6::2], upd.gn.groups,
-                                                 params[3], params[4], upd.gn.epsilon)
-        ctx.rows_saved = saved if any(ctx.needs_input_grad) else None
+        outs, rows = ops.painn_update_train_fwd(x_a, x_at, x_v, x_vt, params[:3], params[5::2], params[6::2], upd.gn.groups,
+                                                params[3], params[4], upd.gn.epsilon)
+        ctx.save_for_backward(x_a, x_at, x_v, x_vt, *params, *(rows if any(ctx.needs_input_grad) else ()))
         ctx.set_materialize_grads(False)
         return tuple(outs)
 
     @staticmethod
     def backward(ctx, g_a, g_v, g_at=None, g_vt=None):
         upd, need = ctx.upd, list(ctx.needs_input_grad)
-        x_a, x_at, x_v, x_vt, *params = ctx.saved_tensors
+        x_a, x_at, x_v, x_vt, *saved = ctx.saved_tensors
+        params, rows = saved[:11], saved[11:]
         if all(g is None for g in (g_a, g_v, g_at, g_vt)):
             return (None,) * len(need)
         if torch.is_grad_enabled():
@@ -843,7 +844,7 @@ class _PainnUpdate(torch.autograd.Function):
         g_a, g_v = zeros(g_a, x_a), zeros(g_v, x_v)
         if x_vt is not None:
             g_at, g_vt = zeros(g_at, x_a), zeros(g_vt, x_v)
-        g_x, d_params = ops.painn_update_train_bwd(g_a, g_at, g_v, g_vt, params[5::2], upd.gn.groups, params[3], ctx.rows_saved)
+        g_x, d_params = ops.painn_update_train_bwd(g_a, g_at, g_v, g_vt, params[5::2], upd.gn.groups, params[3], rows)
         grads = list(g_x) + list(d_params)
         return (None,) + tuple(g if nd else None for g, nd in zip(grads, need[1:]))
 

@@ -963,6 +963,43 @@ def test_painn_layers_of_values_and_tangents(pkg, B, N, n, n_rbf, degree):
         _close(a, b, f"gradient {k}", 1.6e-5)
 
 
+@pytest.mark.parametrize("r_grad", [False, True])
+def test_what_the_fused_painn_layers_keep_passes_the_saved_tensor_hooks(pkg, r_grad):
+    """Message (its filter from the grid, or the MLP on every edge where the edge vectors are differentiated) and Update keep
+    the rows of their hidden layers through save_for_backward: hooks such as save_on_cpu see them, a graph that has been
+    backpropagated holds none of them, and the gradients are the same ones."""
+    painn = importlib.import_module("learned-dynamics_amd.painn")
+    gl = importlib.import_module("learned-dynamics_amd.graph_layers")
+    torch.manual_seed(0x947)
+    n, N, E = 32, 60, 2400 if r_grad else 9000
+    src, dst = torch.sort(torch.randint(0, N, (E,))).values, torch.randint(0, N, (E,))
+    graph = gl.Graph(src.cuda(), dst.cuda(), None, 1, N)
+    msg, upd = painn.Message(5.0, n, 16).cuda(), painn.Update(n).cuda()
+    x_a, x_v, r = torch.randn(1, N, n).cuda(), torch.randn(1, N, n, 3).cuda(), torch.randn(E, 3).cuda()
+    leaves = [x_a.requires_grad_(), x_v.requires_grad_()] + ([r.requires_grad_()] if r_grad else [])
+    leaves += list(msg.parameters()) + list(upd.parameters())
+
+    def loss():
+        da, dv = msg(graph, x_a, x_v, r)
+        ya, yv = upd(x_a + da, x_v + dv)
+        return (ya ** 2).sum() + (yv ** 2).sum()
+
+    want = torch.autograd.grad(loss(), leaves)
+    packed = []
+
+    def pack(t):
+        packed.append(tuple(t.shape))
+        return t.detach().cpu()
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()):
+        value = loss()
+    got = torch.autograd.grad(value, leaves)
+    for mlp, rows in ((msg.mlp_actv, N), (upd.mlp, N)) + (((msg.mlp_dist, E),) if r_grad else ()):
+        assert packed.count((rows, mlp.layers[0].out_features)) >= 4, "two hidden layers, before and after the activation"
+    for k, (a, b) in enumerate(zip(got, want)):
+        torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5 * float(b.abs().max()), msg=f"gradient {k}")
+
+
 @pytest.mark.parametrize("n,rows,N,E,seed", [(16, 4, 3, 40, 0), (32, 64, 50, 3000, 1), (128, 512, 700, 20000, 2), (256, 512, 33, 5, 3),
                                             (128, 512, 40, 500000, 4)])
 def test_gradients_of_the_message_from_its_grid(pkg, ops, n, rows, N, E, seed):
