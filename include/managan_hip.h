@@ -564,6 +564,24 @@ int mg_bee_edge_filters_fwd(const float* enc, const float* rh, long E, int chan,
 int mg_bee_edge_filters_bwd(const float* enc, const float* rh, const float* g_v, const float* g_d, long E, int chan,
                             float* d_enc, float* d_rh, mg_stream_t stream);
 
+/* Gradients of the 13 message products of Messages (archs/diffuser_atoms15.py:238-253; chan a multiple of 64:
+ * mg_bee_message_grad_supported) for the operands l_0 (n_rows, chan), l_1 (.., 3), l_2 (.., 3, 3), read at dst[e], and for enc
+ * (E, chan) and rh (E, 3), which the edge filters enc, enc rh, enc rh (x) rh are made of.  dy, in the order of mg_bee_fwd:
+ * the products 000, 110, 220 hold E rows, the others n_src rows, the gradient of their sums over the edges of a source node
+ * (row_ptr: the CSR of the edges, which are sorted by source).  dst_row_ptr / perm: the edges sorted by destination.
+ * Outputs are null where not wanted; d_0, d_1, d_2 come together.  Sums run in a fixed order. */
+int mg_bee_message_grad_supported(int chan);   /* returns 0 / 1, not a status */
+int mg_bee_message_grad_workspace_bytes(long E, int chan, int want_left, int want_rh, size_t* bytes);
+typedef struct mg_bee_message_grad {
+    const float *l_0, *l_1, *l_2, *enc, *rh, *dy[13];
+    const int *row_ptr, *dst, *dst_row_ptr, *perm;
+    long E;
+    int n_src, n_rows, chan;
+    void* workspace;
+    float *d_0, *d_1, *d_2, *d_enc, *d_rh;
+} mg_bee_message_grad;
+int mg_bee_message_grad_run(const mg_bee_message_grad* args, mg_stream_t stream);
+
 /* SiLU and its derivatives for the MLPs' training path (nn.SiLU in archs/meanflow_painn8.py:38-51, differentiated up
  * to three times by the meanflow loss, :274-296): out[k] = SiLU^(order)(z[k]) (* mul[k] if mul is not null), order 0..4,
  * n floats, 16-byte aligned.  The reference leaves these derivatives to autograd's elementwise formulas. */

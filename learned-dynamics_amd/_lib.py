@@ -120,6 +120,9 @@ _SIGNATURES = {
     "mg_painn_grid_node_grad": [vp, vp, vp, vp, i32, i64, vp, vp, i32, f32, f32, vp, vp, vp, vp, i32, vp, vp, vp, vp],
     "mg_painn_grid_rows": [vp, i64, i32, f32, vp, vp],
     "mg_painn_grid_table_grad": [vp, vp, vp, vp, i32, i64, vp, i32, f32, f32, vp, vp, vp, vp, i32, vp, vp, vp],
+    "mg_bee_message_grad_supported": [i32],
+    "mg_bee_message_grad_workspace_bytes": [i64, i32, i32, i32, vp],
+    "mg_bee_message_grad_run": [vp, vp],
     "mg_sort_by_key_workspace_bytes": [i64, vp],
     "mg_sort_by_key": [vp, i64, i32, vp, vp, vp, vp],
     "mg_silu_rows_fwd": [vp, i64, i32, i32, vp, vp, vp],

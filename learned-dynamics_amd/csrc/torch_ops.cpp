@@ -1039,6 +1039,70 @@ std::tuple<OptTensor, OptTensor, OptTensor> painn_grid_message_bwd(const at::Ten
     return {d_table, d_actv, d_v};
 }
 
+// gradients of the rank-0/1/2 message products: (l_0, l_1, l_2), enc, rh; see mg_bee_message_grad
+std::tuple<Tensors, OptTensor, OptTensor> bee_message_bwd(const Tensors& left, const at::Tensor& enc, const at::Tensor& rh,
+                                                          const Tensors& dy, const at::Tensor& row_ptr, const at::Tensor& dst,
+                                                          const at::Tensor& dst_row_ptr, const OptTensor& perm, bool want_left,
+                                                          bool want_enc, bool want_rh) {
+    static const int rank_of[13] = {0, 0, 0, 1, 1, 1, 1, 2, 2, 2, 2, 1, 2};
+    TORCH_CHECK(left.size() == 3 && dy.size() == 13, "bee_message_bwd: three operands and 13 gradients expected");
+    check_input(enc, "enc");
+    check_input(rh, "rh");
+    check_input(row_ptr, "row_ptr", at::kInt);
+    check_input(dst, "dst", at::kInt);
+    check_input(dst_row_ptr, "dst_row_ptr", at::kInt);
+    if (perm.has_value()) check_input(*perm, "perm", at::kInt);
+    TORCH_CHECK(enc.dim() == 2 && rh.dim() == 2, "bee_message_bwd: enc (edges, chan) and rh (edges, 3) expected");
+    const int64_t E = enc.size(0), C = enc.size(1), rows = left[0].size(0), n_src = row_ptr.numel() - 1;
+    const int64_t per_rank[3] = {C, 3 * C, 9 * C};
+    TORCH_CHECK(rh.numel() == 3 * E && dst.numel() == E && dst_row_ptr.numel() == rows + 1 && n_src >= 0 &&
+                    (!perm.has_value() || perm->numel() == E),
+                "bee_message_bwd: operand sizes");
+    mg_bee_message_grad a{};
+    for (int k = 0; k < 3; k++) {
+        check_input(left[k], "left operand");
+        TORCH_CHECK(left[k].numel() == rows * per_rank[k], "bee_message_bwd: operand sizes");
+    }
+    for (int k = 0; k < 13; k++) {
+        check_input(dy[k], "gradient of a product");
+        TORCH_CHECK(dy[k].numel() == (rank_of[k] ? n_src : E) * per_rank[rank_of[k]], "bee_message_bwd: gradient sizes");
+        a.dy[k] = fp(dy[k]);
+    }
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(enc.device());
+    Tensors d_left;
+    if (want_left)
+        for (const at::Tensor& t : left) d_left.push_back(floats(t, t.sizes()));
+    at::Tensor d_enc, d_rh;
+    if (want_enc) d_enc = floats(enc, enc.sizes());
+    if (want_rh) d_rh = floats(rh, rh.sizes());
+    size_t bytes = 0;
+    check(mg_bee_message_grad_workspace_bytes(E, (int)C, want_left, want_rh, &bytes));
+    at::Tensor ws = bytes_like(enc, bytes);
+    a.l_0 = fp(left[0]);
+    a.l_1 = fp(left[1]);
+    a.l_2 = fp(left[2]);
+    a.enc = fp(enc);
+    a.rh = fp(rh);
+    a.row_ptr = row_ptr.data_ptr<int>();
+    a.dst = dst.data_ptr<int>();
+    a.dst_row_ptr = dst_row_ptr.data_ptr<int>();
+    a.perm = perm.has_value() ? perm->data_ptr<int>() : nullptr;
+    a.E = E;
+    a.n_src = (int)n_src;
+    a.n_rows = (int)rows;
+    a.chan = (int)C;
+    a.workspace = ws.data_ptr();
+    if (want_left) {
+        a.d_0 = fp(d_left[0]);
+        a.d_1 = fp(d_left[1]);
+        a.d_2 = fp(d_left[2]);
+    }
+    a.d_enc = want_enc ? fp(d_enc) : nullptr;
+    a.d_rh = want_rh ? fp(d_rh) : nullptr;
+    check(mg_bee_message_grad_run(&a, stream_of(enc)));
+    return {d_left, want_enc ? OptTensor(d_enc) : OptTensor(), want_rh ? OptTensor(d_rh) : OptTensor()};
+}
+
 }  // namespace
 
 void register_ops(pybind11::module_& m) {
@@ -1057,6 +1121,7 @@ void register_ops(pybind11::module_& m) {
     m.def("painn_message_edges", &painn_message_edges);
     m.def("sort_by_key", &sort_by_key);
     m.def("painn_grid_message_bwd", &painn_grid_message_bwd);
+    m.def("bee_message_bwd", &bee_message_bwd);
     m.def("mlp_silu_fwd", &mlp_silu_fwd);
     m.def("mlp_silu_bwd", &mlp_silu_bwd);
     m.def("edge_encode_fwd", &edge_encode_fwd);

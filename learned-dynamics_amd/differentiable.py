@@ -905,9 +905,8 @@ class _MessageProducts(torch.autograd.Function):
     inference kernel of the layer (mg_bee_message: filters formed in registers, node rows gathered at the destination,
     products summed over the edges of a node; only the three scalar products are stored per edge) when `enc_source`
     = (the 8 radial functions, weight and bias of the encoding linear) is given, else the indexed product kernel and
-    segment sums.  Backward: the filters are recomputed, the two gradient kernels read the node operands at the
-    destination and the gradients of the summed products at the source through the indices, and the filters' adjoint
-    folds the three filter gradients into those of enc and rh.  A recorded backward pass (create_graph=True)
+    segment sums.  Backward: one kernel walks the edges of a source node with the gradients of its sums in registers and
+    yields the gradients of enc and rh and, per edge, of the node operands, which a second one sums by destination.  A recorded backward pass (create_graph=True)
     differentiates the plain formulation instead."""
 
     @staticmethod
@@ -962,21 +961,10 @@ class _MessageProducts(torch.autograd.Function):
                 out = _message_products_plain(*leaves, by_dst, by_src)
                 grads = torch.autograd.grad(out, leaves, dys, create_graph=True)
             return tuple(g if nd else None for g, nd in zip(grads, need)) + (None, None, None)
-        a_node, v_node, d_node, enc, rh = saved
-        dys = [dy.contiguous() for dy in dys]
-        E = enc.size(0)
-        phi_v, phi_d = ops.bee_edge_filters_fwd(enc, rh)
-        d_l = (None, None, None)
-        d_enc = d_rh = None
-        if any(need[:3]):
-            per_edge = ops.bee_bwd_indexed(0, enc, phi_v, phi_d, None, dys, by_src.index, E)
-            d_l = tuple(ops.segment_sum_csr(t, by_dst.row_ptr, by_dst.n_rows, perm=by_dst.perm) if nd else None
-                        for t, nd in zip(per_edge, need[:3]))
-        if need[3] or need[4]:
-            dr_0, dr_1, dr_2 = ops.bee_bwd_indexed(1, a_node, v_node, d_node, by_dst.index, dys, by_src.index, E)
-            d_enc, d_rh = ops.bee_edge_filters_bwd(enc, rh, dr_1, dr_2)
-            d_enc = d_enc + dr_0
-        return (*d_l, d_enc if need[3] else None, d_rh if need[4] else None, None, None, None)
+        *left, enc, rh = saved
+        d_l, d_enc, d_rh = ops.bee_message_bwd(left, enc, rh, [dy.contiguous() for dy in dys], by_src, by_dst, any(need[:3]),
+                                               need[3], need[4])
+        return tuple(d_l[k] if need[k] else None for k in range(3)) + (d_enc, d_rh, None, None, None)
 
 
 def message_products(graph, a_node, v_node, d_node, enc, rh, enc_source=None):

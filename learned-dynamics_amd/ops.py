@@ -575,6 +575,14 @@ def bee_bwd_indexed(side, o_0, o_1, o_2, o_index, dys, dy_index, rows):
     return d
 
 
+def bee_message_bwd(left, enc, rh, dys, by_src, by_dst, want_left, want_enc, want_rh):
+    """Gradients of the 13 products of the node operands `left`, read at the edges' destinations, with the edge filters made
+    of enc (edges, chan) and rh (edges, 3): ([d_l0, d_l1, d_l2] or [], d_enc or None, d_rh or None).  dys: one row per edge
+    for the scalar products, one per source node for the others (their sums over its edges)."""
+    return _ext.bee_message_bwd(list(left), enc, rh, list(dys), by_src.row_ptr, by_dst.index, by_dst.row_ptr, by_dst.perm,
+                                bool(want_left), bool(want_enc), bool(want_rh))
+
+
 def bee_bwl(r_0, r_1, r_2, *dys):
     return _bee_bwd(0, r_0, r_1, r_2, dys)
 

@@ -822,6 +822,44 @@ def test_message_products_with_folded_gathers(pkg):
     assert all(bool(torch.isfinite(t).all()) for t in second)
 
 
+@pytest.mark.parametrize("N,E,C", [(1, 1, 64), (5, 3, 192), (37, 500, 128), (9, 2000, 256), (700, 4096, 64)])
+def test_gradients_of_the_rank012_message_products(pkg, ops, N, E, C):
+    """ops.bee_message_bwd against the products of rank 0-2 differentiated in float64: one edge, one slice of 64 channels and
+    several, a last workgroup that is not full, nodes without edges on either side, odd and even numbers of edges at a
+    destination; each gradient alone gives what all together give.  Tolerance: the node gradients are sums over an edge's 63 and
+    a destination's terms, those of rh over an edge's 63 terms and all channels: 2^-24 sqrt(terms) of the largest entry, with a factor 8."""
+    gl = importlib.import_module("learned-dynamics_amd.graph_layers")
+    g = torch.Generator().manual_seed(0x947 + E)
+    src = torch.sort(torch.randint(0, N, (E,), generator=g)).values
+    dst = torch.randint(0, max(1, N - 1), (E,), generator=g)
+    rnd = lambda *shape: torch.randn(*shape, generator=g)
+    graph = gl.Graph(src.cuda(), dst.cuda(), None, 1, N)
+    left, enc, rh = [rnd(N, C, *([3] * k)) for k in range(3)], rnd(E, C), rnd(E, 3)
+    dys = [rnd(N if k else E, C, *([3] * k)) for k in (0, 0, 0, 1, 1, 1, 1, 2, 2, 2, 2, 1, 2)]
+    xs = [t.double().requires_grad_() for t in (*left, enc, rh)]
+    phi_v = xs[3][..., None] * xs[4][:, None]
+    phi_d = phi_v[..., None] * xs[4][:, None, None]
+    prods = OP.bee(*[t[dst] for t in xs[:3]], xs[3], phi_v, phi_d)
+    # (the gradient of an edge's product is the gradient of its source node's sum)
+    total = sum((p * (d.double() if d.dim() == 2 else d.double()[src])).sum() for p, d in zip(prods, dys))
+    ref = torch.autograd.grad(total, xs)
+    args = ([t.cuda() for t in left], enc.cuda(), rh.cuda(), [t.cuda() for t in dys], graph.by_src, graph.by_dst)
+    d_left, d_enc, d_rh = ops.bee_message_bwd(*args, True, True, True)
+    for name, x, y, terms in zip(("l_0", "l_1", "l_2", "enc", "rh"), (*d_left, d_enc, d_rh), ref, (63 * E, 63 * E, 63 * E, 63, 63 * C)):
+        err = float((x.cpu().double() - y).abs().max() / y.abs().max())
+        assert err <= 8 * 2 ** -24 * terms ** 0.5, f"{name}: {err:.3g}"
+    alone = ops.bee_message_bwd(*args, True, False, False)
+    assert all(torch.equal(a, b) for a, b in zip(alone[0], d_left)) and alone[1] is None and alone[2] is None
+    assert torch.equal(ops.bee_message_bwd(*args, False, True, False)[1], d_enc)
+    assert torch.equal(ops.bee_message_bwd(*args, False, False, True)[2], d_rh)
+    if ops.bee_indexed_supported(C):                                    # the same one edge at a time
+        phi = ops.bee_edge_filters_fwd(enc.cuda(), rh.cuda())
+        per_edge = ops.bee_bwd_indexed(0, enc.cuda(), *phi, None, args[3], graph.by_src.index, E)
+        for x, y, z in zip(per_edge, d_left, ref):
+            x = torch.zeros_like(z).index_add_(0, dst, x.cpu().double())
+            assert float((x - y.cpu()).abs().max()) <= 8 * 2 ** -24 * (63 * E) ** 0.5 * float(z.abs().max())
+
+
 @pytest.mark.parametrize("E,C", [(300, 256), (17, 40), (1000, 64), (5, 700)])
 def test_edge_filters_against_broadcasting_arithmetic(pkg, E, C):
     """phi_v = enc (x) rh and phi_d = enc (x) rh (x) rh of Messages (archs/diffuser_atoms15.py:241-243) as one kernel:
