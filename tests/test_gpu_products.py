@@ -148,6 +148,22 @@ def test_tensor_prods_one_launch(ops, lro):
     assert_parity(y, ref32, ref64, what=f"tensor_prods {lro}")
 
 
+@pytest.mark.parametrize("lro", [(1, 1, 0), (0, 1, 1), (2, 1, 1), (1, 1, 2), (2, 2, 2)])
+@pytest.mark.parametrize("rows,dims", [(1, (64, 64, 64, 64)), (17, (32, 32, 32, 32)), (33, (16, 32, 48, 16)), (130, (32, 16, 80, 96)),
+                                       (40, (48, 64, 32, 64)), (8193, (32, 16, 32, 16)), (49153, (16, 16, 64, 16))])
+def test_tensor_prods_few_rows(ops, lro, rows, dims):
+    """The kernels whose waves share 16 rows: four waves (64 inner channels and up: 64, 80 leave a last trip with one wave at
+    work) and two (32, 48), fewer output tiles than waves and more, a second grid row of output tiles, a last group past the end
+    of the rows; and the first row counts that the other kernel takes (8193 and 49153).  (dims: l, r, rank, o)"""
+    from parity import assert_parity
+    x_l, x_r, W_l, W_r, W_o = _tp_case(lro, rows, dims, 300 + rows + sum(lro))
+    assert ops.tensor_prods_supported(*lro, *dims)
+    y = ops.tensor_prods(*lro, W_l.cuda(), W_r.cuda(), W_o.cuda(), x_l.cuda(), x_r.cuda())
+    ref32 = OP.tensor_prods(*lro, W_l, W_r, W_o, x_l, x_r)
+    ref64 = OP.tensor_prods(*lro, W_l.double(), W_r.double(), W_o.double(), x_l.double(), x_r.double())
+    assert_parity(y, ref32, ref64, what=f"tensor_prods {lro}, {rows} rows, {dims}")
+
+
 def test_tensor_prods_module_routes_and_agrees(ops):
     """TensorProds.forward takes the one-launch kernel when nothing asks for a gradient and the three-step path
     otherwise; both agree with the oracle; strided weights (a transposed view) and leading batch axes are honoured;
