@@ -67,20 +67,21 @@ struct RowFromMemory {
 // columns, i = 8 (q / 4) + 4 (lane / 32) + q % 4: the split-fp16 row-streaming main loop with W as the first
 // matrix operand.  a_src(v, k0) delivers the lane's 16 values of x for chunk k0 (two chunks ahead of their use);
 // lds: 2 * kFBufW bytes; all waves of the workgroup call it together, and the W buffers are free again when it
-// returns.
-template <typename ASrc>
-__device__ __forceinline__ void wfirst_gemm_tile(floatx16 (&acc)[kFNI], const _Float16* __restrict__ Wp,
+// returns.  NI: blocks of 32 columns in the tile (2 * NI * 4096 bytes of lds).
+template <int NI = kFNI, typename ASrc>
+__device__ __forceinline__ void wfirst_gemm_tile(floatx16 (&acc)[NI], const _Float16* __restrict__ Wp,
                                                  long plane_elems, int n0, const ASrc& a_src, int I,
                                                  float sx, unsigned char* lds) {
-    constexpr int THREADS = kFThreads, kPlaneW = kFPlaneW, kBufW = kFBufW;
-    constexpr int kPer = 8 * kFTN / THREADS;                 // 16-byte pieces of W per thread and chunk
+    constexpr int THREADS = kFThreads, TN = 32 * NI, kPlaneW = TN * 64, kBufW = 2 * kPlaneW;
+    constexpr int kPer = 8 * TN / THREADS;                   // 16-byte pieces of W per thread and chunk
+    static_assert(8 * TN % THREADS == 0, "whole pieces per thread");
     const int tid = threadIdx.x;
     const _Float16* wsrc[kPer];
     int wdst[kPer];
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
         const int q = tid + THREADS * j;
-        const int plane = q / (4 * kFTN), i = q % (4 * kFTN);
+        const int plane = q / (4 * TN), i = q % (4 * TN);
         wsrc[j] = Wp + plane * plane_elems + packed_piece(n0, i, I);
         wdst[j] = plane * kPlaneW + 16 * i;
     }
@@ -113,7 +114,7 @@ __device__ __forceinline__ void wfirst_gemm_tile(floatx16 (&acc)[kFNI], const _F
 #pragma unroll
         for (int s = 0; s < 2; s++)
 #pragma unroll
-            for (int ni = 0; ni < kFNI; ni++) {
+            for (int ni = 0; ni < NI; ni++) {
                 const halfx8 bh = *reinterpret_cast<const halfx8*>(buf + b_off + 2048 * ni + 1024 * s);
                 const halfx8 bl = *reinterpret_cast<const halfx8*>(buf + kPlaneW + b_off + 2048 * ni + 1024 * s);
                 // W first: D[i][j] with i the filter column in the block and j the edge
@@ -121,7 +122,7 @@ __device__ __forceinline__ void wfirst_gemm_tile(floatx16 (&acc)[kFNI], const _F
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bl, ah[s], acc[ni], 0, 0, 0);
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bh, ah[s], acc[ni], 0, 0, 0);
             }
-        order_chunk<kFNI>();
+        order_chunk<NI>();
     };
 
     unsigned char* buf0 = lds;
@@ -367,8 +368,8 @@ painn_filter_message_kernel(const _Float16* __restrict__ Wp, const float* __rest
 // y = act(x W^T + bias) for rows sorted by segment (seg[row] ascending), reduced over the rows of each segment
 // in the epilogue: out[s] = scale * sum_{rows of s} y[row].  Same tile, same slots A / B per block of 32 rows
 // and same finishing pass as the message kernel above; y itself is written only when STORE_Y is set
-// (coalesced, from the LDS slice the reduction reads anyway).
-template <int ACT, bool STORE_Y>
+// (coalesced, from the LDS slice the reduction reads anyway).  NI: the tile's columns / 32.
+template <int ACT, bool STORE_Y, int NI>
 __global__ void __launch_bounds__(64 * kFW)
 linear_rowsum_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restrict__ w_inv,
                            const float* __restrict__ bias, const float* __restrict__ X,
@@ -376,9 +377,9 @@ linear_rowsum_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restr
                            const int* __restrict__ seg, float* __restrict__ slots, long n_blocks, float scale,
                            float* __restrict__ Y, float* __restrict__ out, int tiles_n, long tiles_total,
                            float bound_mul, float bound_add) {
-    constexpr int kSlice = kFSlice, kRed = kFRed;
+    constexpr int kSlice = kFSlice, kRed = kFRed, TN = 32 * NI;
     __shared__ __attribute__((aligned(16))) unsigned char lds[kFLds];
-    __shared__ __attribute__((aligned(16))) float wb[2 * kFTN];   // the tile's 1 / weight scale, then its bias
+    __shared__ __attribute__((aligned(16))) float wb[2 * TN];   // the tile's 1 / weight scale, then its bias
 
     const long bid = blockIdx.x;
     const long per_xcd = (tiles_total + 7) / 8;
@@ -389,12 +390,12 @@ linear_rowsum_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restr
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int m = lane & 31, g = lane >> 5;
-    const int n0 = tile_n * kFTN;
+    const int n0 = tile_n * TN;
     const long plane_elems = (long)O * I;
 
-    floatx16 acc[kFNI];
+    floatx16 acc[NI];
 #pragma unroll
-    for (int ni = 0; ni < kFNI; ni++)
+    for (int ni = 0; ni < NI; ni++)
 #pragma unroll
         for (int q = 0; q < 16; q++) acc[ni][q] = 0.f;
 
@@ -411,11 +412,11 @@ linear_rowsum_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restr
         sx = pow2_scale(amax, &isx);
     }
     const int my_seg = seg[ld_row];
-    if (tid < kFTN) {
+    if (tid < TN) {
         wb[tid] = w_inv[n0 + tid];
-        wb[kFTN + tid] = bias ? bias[n0 + tid] : 0.f;
+        wb[TN + tid] = bias ? bias[n0 + tid] : 0.f;
     }
-    wfirst_gemm_tile(acc, Wp, plane_elems, n0, RowFromMemory{xrow, I}, I, sx, lds);
+    wfirst_gemm_tile<NI>(acc, Wp, plane_elems, n0, RowFromMemory{xrow, I}, I, sx, lds);
 
     const float keep = my_row < R ? 1.f : 0.f;               // rows past the end add nothing
     const long rows_left = R - block * 32;
@@ -429,7 +430,7 @@ linear_rowsum_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restr
     float* slot_b = slots + (n_blocks + block) * O;
 
 #pragma unroll
-    for (int pass = 0; pass < 4; pass++) {
+    for (int pass = 0; pass < NI / 2; pass++) {
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const int ni = 2 * pass + h;
@@ -437,7 +438,7 @@ linear_rowsum_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restr
             for (int qq = 0; qq < 4; qq++) {
                 const int cl = 32 * ni + 8 * qq + 4 * g;      // column in the tile
                 const float4 iw = *reinterpret_cast<const float4*>(wb + cl);
-                const float4 bv = *reinterpret_cast<const float4*>(wb + kFTN + cl);
+                const float4 bv = *reinterpret_cast<const float4*>(wb + TN + cl);
                 float4 v;
                 v.x = keep * activate_c<ACT>(acc[ni][4 * qq + 0] * isx * iw.x + bv.x);
                 v.y = keep * activate_c<ACT>(acc[ni][4 * qq + 1] * isx * iw.y + bv.y);
@@ -775,15 +776,31 @@ int mg_tensor_linear_f16x2_rowsum_scaled_bound(const void* packed_W, const float
     if (rows > 0) {
         MG_REQUIRE(x && x_rowmax && seg && workspace && aligned16(x) && aligned16(workspace) && (!y || aligned16(y)),
                    "mg_tensor_linear_f16x2_rowsum: null or unaligned row operand");
-        const int tiles_n = dim_out / kFTN;
-        const long tiles_total = ceil_div(rows, kFTM) * tiles_n;
+        // Column tile by the cost of the plain linear at few rows (tensor_linear_f16x2.hip, choose_tile): rounds of 256
+        // workgroups times 5 us + chunks x (1 + ni / 4) us.  30 200 rows, 768 -> 256: 118 tiles of
+        // 256 columns leave half the chip idle, 81 us; 236 of 128 columns 56 us.
+        const long tiles_m = ceil_div(rows, kFTM), chunks = ceil_div(dim_in, 32);
+        int ni = 8;
+        long best = -1;
+        for (int k = 8; k >= 2; k >>= 1) {
+            const long cost = ceil_div(tiles_m * (dim_out / (32 * k)), 256) * (20 + chunks * (4 + k));
+            if (best < 0 || cost < best) { best = cost; ni = k; }
+        }
+        const int tiles_n = dim_out / (32 * ni);
+        const long tiles_total = tiles_m * tiles_n;
         const _Float16* planes = static_cast<const _Float16*>(packed_W);
         const float* w_inv = reinterpret_cast<const float*>(planes + 2L * dim_out * dim_in);
         const long grid = 8 * ceil_div(tiles_total, 8);
         MG_REQUIRE(grid < (1L << 31), "mg_tensor_linear_f16x2_rowsum: too many tiles");
         float* slots = static_cast<float*>(workspace);
 #define MG_ROWSUM_LAUNCH(A, S)                                                                                       \
-    linear_rowsum_f16x2_kernel<A, S><<<dim3((unsigned)grid), dim3(64 * kFW), 0, s>>>(                                \
+    do {                                                                                                             \
+        if (ni == 8) MG_ROWSUM_TILE(A, S, 8);                                                                        \
+        else if (ni == 4) MG_ROWSUM_TILE(A, S, 4);                                                                   \
+        else MG_ROWSUM_TILE(A, S, 2);                                                                                \
+    } while (0)
+#define MG_ROWSUM_TILE(A, S, NI_)                                                                                       \
+    linear_rowsum_f16x2_kernel<A, S, NI_><<<dim3((unsigned)grid), dim3(64 * kFW), 0, s>>>(                                \
         planes, w_inv, bias, x, x_rowmax, x_rowmax_parts, x_rowmax_stride, rows, dim_in, dim_out, seg, slots, n_blocks, \
         scale, y, out, tiles_n, tiles_total, bound_mul, bound_add)
         if (y) {
@@ -795,6 +812,7 @@ int mg_tensor_linear_f16x2_rowsum_scaled_bound(const void* packed_W, const float
             else if (act == 2) MG_ROWSUM_LAUNCH(2, false);
             else MG_ROWSUM_LAUNCH(0, false);
         }
+#undef MG_ROWSUM_TILE
 #undef MG_ROWSUM_LAUNCH
         if (int st = check_launch("linear_rowsum_f16x2_kernel")) return st;
     }

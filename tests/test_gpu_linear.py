@@ -366,6 +366,24 @@ def test_linear_with_row_sums_in_the_epilogue(ops, dim_in, dim_out, act, kind, w
     assert not bool(out[(lengths == 0).cuda()].any())
 
 
+@pytest.mark.parametrize("rows,dim_in,dim_out", [(4500, 96, 512), (20001, 64, 256), (70000, 64, 256)])
+def test_row_sums_in_the_epilogue_at_every_tile_width(ops, rows, dim_in, dim_out):
+    """Row counts for which the rule takes tiles of 64, 128 and 256 columns: the rows bit for bit those of the plain linear (an
+    element's order of summation does not depend on the tile), the sums to fp32 rounding."""
+    g = torch.Generator().manual_seed(rows)
+    n_seg = rows // 16
+    seg = torch.sort(torch.randint(0, n_seg, (rows,), generator=g)).values
+    x = torch.randn(rows, dim_in, generator=g).cuda()
+    W, b = (torch.randn(dim_out, dim_in, generator=g) / dim_in ** 0.5).cuda(), torch.randn(dim_out, generator=g).cuda()
+    row_ptr, bound = ops.segment_row_ptr(seg.int().cuda(), n_seg), ops.row_absmax(x)
+    args = (W, x, bound, row_ptr, seg.int().cuda(), n_seg)
+    out, y = ops.tensor_linear_f16x2_rowsum(*args, bias=b, act=2, want_rows=True)
+    assert torch.equal(y, ops.tensor_linear_f16x2(W, x, bound, bias=b, act=2))
+    assert torch.equal(ops.tensor_linear_f16x2_rowsum(*args, bias=b, act=2)[0], out)
+    z = torch.nn.functional.leaky_relu(x.cpu().double() @ W.cpu().double().T + b.cpu().double(), 0.1)
+    _check(out, lambda dt: torch.zeros(n_seg, dim_out, dtype=dt).index_add_(0, seg, z.to(dt)), f"row sums, {rows} rows")
+
+
 @pytest.mark.parametrize("inds,rows,dim_in,dim_out", [(2, 8000, 16, 64), (1, 22000, 40, 96), (1, 30000, 64, 256), (1, 25000, 70, 64)])
 def test_component_major_output_from_reference_layout_at_many_rows(ops, inds, rows, dim_in, dim_out):
     """x in the reference layout (rows, chan, 3..), y component-major (rows, 3^inds, chan_out): at many rows
