@@ -187,6 +187,13 @@ __global__ void __launch_bounds__(256) components_to_rows_kernel(const float* __
     if (live && k0 == 0) rowmax[out_row] = mx;
 }
 
+// a barrier that orders LDS only: __syncthreads() would also wait for the stores to memory
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 template <int WAVES, int NI>
 __global__ void __launch_bounds__(64 * WAVES)
 linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restrict__ w_inv, const float* __restrict__ X,
@@ -198,7 +205,10 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
     constexpr int kPlaneW = TN * 64, kBufW = 2 * kPlaneW;
     constexpr int kPieces = 8 * TN;                          // 16-byte pieces of W per chunk (2 planes x TN rows x 4)
     constexpr int kPer = (kPieces + THREADS - 1) / THREADS;  // per thread
-    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kBufW];
+    // component rows of nine leave through LDS in this tile only (epilogue_runs): 32 columns of the tile's rows
+    constexpr bool kRuns = WAVES == 4 && NI == 2;
+    constexpr int kStage = kRuns ? 4 * 32 * (TM + 2 * 9) : 0;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kBufW > kStage ? 2 * kBufW : kStage];
     __shared__ float inv_sx[TM];
 
     const long bid = blockIdx.x;
@@ -378,6 +388,37 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
             }
         }
     };
+    // The same for nine components: a lane's values lie 36 bytes from its neighbours', so that every store of a wave would
+    // write four bytes here and there of dozens of lines.  32 columns at a time are put in order in LDS (the W buffers are done
+    // with) and leave in runs.  73 728 rows x 32 -> 256: 65 us stored directly, whatever the tile; 40 us in runs from this
+    // tile, 62 from 256 x 256 (one workgroup per CU, whose passes wait for each other).  With three components direct stores
+    // are faster: 15.6 against 17.7 us for 24 576 x 64 -> 256.
+    auto epilogue_runs = [&](auto t_tag) {
+        constexpr int T = decltype(t_tag)::value;
+        float* stage = reinterpret_cast<float*>(lds);
+        const long row_lo = r0 / T;
+        const int first = (int)(r0 - row_lo * T);                    // the tile's rows are first .. first + TM - 1 of row_lo's
+        const int count = ((first + TM - 1) / T + 1) * (32 * T);
+        const int end = R - r0 < TM ? first + (int)(R - r0) : first + TM;
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++) {
+            const float iw = w_inv[n0 + ni * 32 + m];
+#pragma unroll
+            for (int q = 0; q < 16; q++) {
+                const int rl = wave * 32 + 8 * (q / 4) + 4 * g + (q % 4), row = (first + rl) / T;
+                stage[row * (32 * T) + m * T + (first + rl - row * T)] = acc[ni][q] * inv_sx[rl] * iw;
+            }
+            lds_barrier();
+            for (int e = tid; e < count; e += THREADS) {
+                const int row = e / (32 * T), w = e - row * (32 * T), rr = row * T + w % T;
+                if (rr >= first && rr < end) {
+                    float* yp = Y + ((row_lo + row) * O + n0 + ni * 32) * T + w;
+                    *yp = accumulate ? stage[e] + *yp : stage[e];
+                }
+            }
+            lds_barrier();
+        }
+    };
     if (full_cols && out_T == 1) {
         constexpr std::integral_constant<int, 0> kNone{};
         constexpr std::integral_constant<int, 1> kSilu{};
@@ -395,7 +436,11 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
         return;
     }
     if (full_cols && act == 0 && bias == nullptr && out_T == 3) { epilogue_comps(std::integral_constant<int, 3>{}); return; }
-    if (full_cols && act == 0 && bias == nullptr && out_T == 9) { epilogue_comps(std::integral_constant<int, 9>{}); return; }
+    if (full_cols && act == 0 && bias == nullptr && out_T == 9) {
+        if constexpr (kRuns) epilogue_runs(std::integral_constant<int, 9>{});
+        else epilogue_comps(std::integral_constant<int, 9>{});
+        return;
+    }
 
     // ---- general path: partial column tiles, or components with bias / activation
     float rmax[16];
@@ -784,7 +829,10 @@ int mg_tensor_linear_f16x2_run(const mg_f16x2_linear* args, mg_stream_t stream) 
 #undef MG_SPLITK
         return check_launch("mg_tensor_linear_f16x2");
     }
-    const Shape sh = choose_shape(a.rows, a.dim_in, a.dim_out);
+    Shape sh = choose_shape(a.rows, a.dim_in, a.dim_out);
+    // nine components and a short reduction: bound by the stores, in runs out of this tile (18 432 x 32 -> 256 17 against 19 us,
+    // 73 728 rows 40 against 65); longer reductions keep the tile that re-reads x least
+    if (a.out_comps == 9 && a.dim_in <= 64 && a.dim_out % 64 == 0 && a.act == 0 && a.bias == nullptr) sh = Shape{2, 4};
 #define MG_F16X2_LAUNCH(WV, N)                                                                                             \
     return launch<WV, N>(planes, w_inv, a.x, a.x_rowmax, a.x_rowmax_parts, a.x_rowmax_stride, a.x_rows_per_bound, a.rows,  \
                          a.dim_in, a.dim_out, O_pad, a.bias, a.act, a.accumulate, a.y, a.y_rowmax, a.out_comps,            \

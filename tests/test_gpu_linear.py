@@ -405,6 +405,36 @@ def test_component_major_output_from_reference_layout_at_many_rows(ops, inds, ro
     _check(small, lambda dt: ref(dt)[:500], "component-major output, generic kernel")
 
 
+@pytest.mark.parametrize("rows,dim,comps,pad", [(1, 5, 3, 32), (3, 40, 9, 64), (1030, 256, 9, 256), (4100, 16, 9, 32), (5000, 128, 3, 128),
+                                                (2, 250, 70, 256)])
+def test_components_to_rows(pkg, rows, dim, comps, pad):
+    """One plain row per (row, component), zero-padded, and its largest magnitude, bit for bit: rows of half a wave to four
+    pieces, channel counts that are no multiple of four, a last workgroup that is not full."""
+    L = importlib.import_module("learned-dynamics_amd._lib")
+    x = torch.randn(rows, dim, comps, generator=torch.Generator().manual_seed(rows + dim)).cuda()
+    y, m = torch.full((rows * comps, pad), 7., device="cuda"), torch.full((rows * comps,), 7., device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    L.check(L.load().mg_components_to_rows(x.data_ptr(), rows, dim, comps, pad, y.data_ptr(), m.data_ptr(), stream))
+    want = torch.nn.functional.pad(x.transpose(1, 2), (0, pad - dim)).reshape(rows * comps, pad)
+    assert torch.equal(y, want) and torch.equal(m, want.abs().amax(1))
+
+
+@pytest.mark.parametrize("inds,rows,dim_in,dim_out", [(1, 321, 64, 256), (1, 1000, 40, 128), (2, 117, 32, 256), (2, 8200, 16, 256), (2, 300, 64, 96)])
+def test_component_output_in_runs(ops, inds, rows, dim_in, dim_out):
+    """Reference layout in and out through the plain-row kernels: tiles that begin and end inside a row's components, nine of
+    them in runs (short reductions, whole tiles of 64 columns) and otherwise, and accumulation, against float64."""
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, dim_in, *([3] * inds), generator=g).cuda()
+    W = (torch.randn(dim_out, dim_in, generator=g) / dim_in ** 0.5).cuda()
+    ref = lambda dt: torch.einsum("oi,bit->bot", W.cpu().to(dt), x.cpu().to(dt).reshape(rows, dim_in, -1)).reshape(rows, dim_out, *([3] * inds))
+    y = ops.tensor_linear_fwd(inds, W, x)
+    _check(y, ref, f"components {rows} x {dim_in} -> {dim_out}")
+    rows2 = x.reshape(rows, dim_in, -1).transpose(1, 2).reshape(-1, dim_in).contiguous()
+    if dim_in % 32 == 0 and dim_in >= 64:
+        y2 = ops.tensor_linear_f16x2(W, rows2, ops.row_absmax(rows2), out_comps=3 ** inds, out=y.clone(), accumulate=True)
+        _check(y2.reshape(y.shape), lambda dt: y.cpu().to(dt) + ref(dt), "accumulated")
+
+
 def test_linear_with_row_sums_edge_cases(ops):
     W = torch.randn(256, 64).cuda()
     row_ptr = torch.zeros(11, dtype=torch.int32, device="cuda")
