@@ -145,11 +145,13 @@ __global__ void __launch_bounds__(1024) grid_node_grad_kernel(
         const float sA = sum_over_slots(A, lane), sB = sum_over_slots(B, lane);
         const int c = sub >> 2, q = sub & 3;
         const long ch = slice * kSliceChan + 4 * l4 + c, row4 = node * 4L * n + ch;
-        const float vq = q < 3 ? v[(node * n + ch) * 3 + q] : 0.f;
+        const bool edges = lo < hi;                           // (a node without edges has gradient zero whatever it holds)
+        const float vq = edges && q < 3 ? v[(node * n + ch) * 3 + q] : 0.f;
+        const float a0 = edges ? actv[row4] : 0.f, a1 = edges ? actv[row4 + n] : 0.f;
         float s0 = vq * sA, s1 = vq * sB;                     // v . M0, v . M1: over the lanes q = 0..2 of the channel
         s0 += __shfl_xor(s0, 4); s1 += __shfl_xor(s1, 4);
         s0 += __shfl_xor(s0, 8); s1 += __shfl_xor(s1, 8);
-        if (d_v && q < 3) d_v[(node * n + ch) * 3 + q] = actv[row4] * sA + actv[row4 + n] * sB;
+        if (d_v && q < 3) d_v[(node * n + ch) * 3 + q] = a0 * sA + a1 * sB;
         if (d_actv) {
             if (q == 3) { d_actv[row4 + 2 * n] = sA; d_actv[row4 + 3 * n] = sB; }
             else if (q < 2) d_actv[row4 + q * n] = q ? s1 : s0;
@@ -187,7 +189,8 @@ __global__ void __launch_bounds__(256) grid_row_grad_kernel(const int* __restric
     long e = lo + 16 * wave + sub;
     float4 ra = make_float4(0.f, 0.f, 0.f, 0.f), rb = ra;
     if (e < hi) { ra = rec[2 * e]; rb = rec[2 * e + 1]; }
-    // (a slot past the end takes part in the matrix instructions with weight zero)
+    // (a slot past the end takes part in the matrix instructions with zeros for both operands: what it read are the rows of some
+    // other edge or of node 0, and zero times an infinity there would be NaN)
     for (long e0 = lo + 16 * wave; e0 < hi; e0 += 64) {
         const bool live = e < hi;
         const long from = min(max((long)__float_as_int(ra.x), 0L), n_nodes - 1), to = min(max((long)__float_as_int(ra.y), 0L), n_nodes - 1);
@@ -221,7 +224,7 @@ __global__ void __launch_bounds__(256) grid_row_grad_kernel(const int* __restric
                                 ((uy * z - uz * y) * vx + (uz * x - ux * z) * vy + (ux * y - uy * x) * vz) * av[1],
                                 (ux * x + uy * y + uz * z) * av[2], gs[c] * av[3]};
 #pragma unroll
-            for (int k = 0; k < 4; k++) acc[4 * k + c] = __builtin_amdgcn_mfma_f32_4x4x1f32(my_w, d[k], acc[4 * k + c], 0, 0, 0);
+            for (int k = 0; k < 4; k++) acc[4 * k + c] = __builtin_amdgcn_mfma_f32_4x4x1f32(my_w, live ? d[k] : 0.f, acc[4 * k + c], 0, 0, 0);
         }
         ra = na; rb = nb;
     }
