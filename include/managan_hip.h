@@ -303,7 +303,8 @@ int mg_tensor_linear_packed(const void* packed_W, const float* x, long rows, int
 /* Mode 2: two-piece fp16 split with per-row power-of-two scales, three fp16 MFMAs per product,
  * fp32 accumulation (a few fp32 ulps per product; half the matrix work of mode 1).
  * mg_linear_f16x2_pack_weight: W -> hi / lo fp16 planes (dim_out rounded up to 256 rows) followed by
- * one fp32 inverse scale per row, in caller-owned memory of mg_linear_f16x2_packed_weight_bytes bytes.
+ * one fp32 inverse scale per row (a NaN where the row holds an infinity or NaN) and one flag per 32 rows,
+ * in caller-owned memory of mg_linear_f16x2_packed_weight_bytes bytes.
  * mg_tensor_linear_f16x2: y = act(x W^T + bias) for plain rows x (rows, dim_in), dim_in % 32 == 0;
  * x_rowmax[(r / x_rows_per_bound) * x_rowmax_stride + p], p < x_rowmax_parts, holds upper bounds of
  * max_i |x[r,i]| (the largest part is used; any bound within a factor 2^14 of the true maximum keeps
@@ -311,7 +312,9 @@ int mg_tensor_linear_packed(const void* packed_W, const float* x, long rows, int
  * components of a node that carries one bound): the y_rowmax output of the call that produced x,
  * mg_row_absmax(x) (one part), or a bound the caller derives from the producing layer's weights.  y_rowmax, if not NULL,
  * receives (rows, mg_tensor_linear_f16x2_rowmax_parts(rows, dim_in, dim_out)) partial row maxima of |y|
- * (out_comps must be 1).  out_comps / accumulate / act as in mg_tensor_linear_packed.
+ * (out_comps must be 1).  out_comps / accumulate / act as in mg_tensor_linear_packed.  Rows whose bound is
+ * infinite or 2^96 and more, and columns whose weights hold an infinity or NaN, are summed in fp32: infinities and NaN
+ * come out as fp32 arithmetic has them; the row maxima emitted there are infinite.
  * Same contraction as tensor_linear (extensions/tensor_ops/tensor_ops.cpp:31-93); packing, scales
  * and row maxima have no counterpart in the reference. */
 int mg_linear_f16x2_packed_weight_bytes(int dim_in, int dim_out, size_t* bytes /* host */);

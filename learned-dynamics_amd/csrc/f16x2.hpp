@@ -12,7 +12,7 @@ typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
 
 
 // power of two s with amax * s in [2^14, 2^15); *inv = 1/s.  amax >= 0; zero, tiny, inf and nan give
-// a finite in-range scale (the products then follow fp16/fp32 arithmetic on their own)
+// a finite in-range scale.  Rows that beyond_split tells apart are not for the fp16 pieces
 __device__ __forceinline__ float pow2_scale(float amax, float* inv) {
     int e = (int)(__float_as_uint(amax) >> 23) & 0xff;
     int se = 268 - e;                   // 127 + 14 - (e - 127)
@@ -21,6 +21,15 @@ __device__ __forceinline__ float pow2_scale(float amax, float* inv) {
     *inv = __uint_as_float((unsigned)(254 - se) << 23);
     return __uint_as_float((unsigned)se << 23);
 }
+
+// A row of x with an infinity (its low piece would be inf - inf), or so large that the scaled sum times 1 / s could overflow
+// before the weight's scale brings it back: the linear kernels take such a row in fp32 (row_in_fp32).  A bound that
+// has overflowed by itself, as one carried through several layers may, only costs time.
+__device__ __forceinline__ bool beyond_split(float amax) { return !(amax < 0x1p96f); }
+// The inverse scale of a weight's row that holds an infinity or NaN: a NaN whose low bits are the exponent of the inverse scale
+// of the row's finite entries.  Every kernel that multiplies by it gives NaN; the linear kernels take the column in fp32.
+__device__ __forceinline__ float mark_weight(float inv) { return __uint_as_float(0x7fc00000u | (__float_as_uint(inv) >> 23)); }
+__device__ __forceinline__ float unmark_weight(float iw) { return iw == iw ? iw : __uint_as_float((__float_as_uint(iw) & 0xffu) << 23); }
 
 struct HalfSplit4 {
     halfx4 hi, lo;
@@ -52,6 +61,26 @@ __host__ __device__ __forceinline__ long packed_index(long o, int k, int I) {
 // of 32); chunk k0 / 32 of the same piece is kPackedChunk * (k0 / 32) = 32 k0 halves further on
 __device__ __forceinline__ long packed_piece(int n0, int i, int I) {
     return ((long)((n0 >> 5) + (i >> 7)) * (I >> 5)) * 1024L + (i & 127) * 8;
+}
+
+// x . w in fp32, k in order, with weight row n put together from its pieces (a weight below 2^-39 of its row's largest is zero
+// there) and iw its inverse scale: what the linear kernels give for the rows and columns marked above.
+__device__ inline float row_in_fp32(const float* x, const _Float16* planes, long plane_elems, long n, int I, float iw) {
+    const float inv = unmark_weight(iw);
+    float sum = 0.f;
+#pragma unroll 1
+    for (int k = 0; k < I; k += 8) {
+        const long at = packed_index(n, k, I);
+        const halfx8 hi = *reinterpret_cast<const halfx8*>(planes + at), lo = *reinterpret_cast<const halfx8*>(planes + plane_elems + at);
+        const float4 x0 = *reinterpret_cast<const float4*>(x + k), x1 = *reinterpret_cast<const float4*>(x + k + 4);
+        const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const float h = (float)hi[j];
+            sum = fmaf(v[j], (fabsf(h) < __builtin_inff() ? h + (float)lo[j] : h) * inv, sum);
+        }
+    }
+    return sum;
 }
 
 // Issue order of one chunk of a tile that is 256 output columns wide (16 fragment pairs, 48 matrix instructions): four

@@ -10,7 +10,8 @@
 // (a W row) into [2^14, 2^15), which removes fp16's narrow exponent range from the picture:
 // an element e of a row with scaled maximum M carries an error of max(2^-22 |e|, 2^-25), i.e.
 // the result is normwise as accurate as the fp32 dot product whenever M >= 1, and the scales
-// are undone exactly in the epilogue.  The row maxima of x come from the kernel that produced
+// are undone exactly in the epilogue.  Rows with an infinity or beyond 2^96, and columns whose weights hold an infinity or NaN,
+// are summed in fp32 by the epilogue (row_in_fp32): the results are those of fp32 arithmetic there too.  The row maxima of x come from the kernel that produced
 // x (this kernel's own epilogue can emit them for its output) or from row_absmax_kernel.
 //
 // Kernel shape (row streaming): a workgroup of WAVES waves owns a tile of 32 WAVES rows x 32 NI
@@ -54,10 +55,16 @@ __device__ __forceinline__ float activate_c(float v) {
     return v;
 }
 
+// behind the inverse scales: per block of 32 output rows whether one of them is marked (mark_weight)
+template <typename F>
+__device__ __forceinline__ auto* marked_blocks(F* inv_scale, int O_pad) {
+    return reinterpret_cast<std::conditional_t<std::is_const_v<F>, const int, int>*>(inv_scale + O_pad);
+}
+
 // Weight planes in fragment order (f16x2.hpp) + 1/scale per row: a workgroup takes a block of 32 output rows (rows past O
 // are zeros), a thread pieces of 8 k of one row, kept in registers between the row maximum (LDS, max of the bit patterns
 // of |w|: any order gives the same) and the split.  One pass over W for I <= kPackRegs * 256.  I_w <= I: columns of W, the
-// others are zeros.
+// others are zeros.  Rows with an infinity or NaN are scaled by their finite entries and marked.
 constexpr int kPackThreads = 1024, kPackRegs = 4;
 // A launch takes up to kPackJobs weights (a training step packs every weight of a layer and its transpose anew: one launch of
 // 10 us per MLP instead of six of 6).
@@ -73,7 +80,7 @@ struct PackJobs {
     int count;
 };
 __global__ void __launch_bounds__(kPackThreads) pack_weight_f16x2_kernel(const PackJobs jobs) {
-    __shared__ unsigned row_max[32];
+    __shared__ unsigned row_max[32], row_odd[32];
     const int tid = threadIdx.x;
     int which = 0;
     while (which + 1 < jobs.count && (int)blockIdx.x >= jobs.job[which + 1].first_block) which++;     // (uniform)
@@ -87,7 +94,7 @@ __global__ void __launch_bounds__(kPackThreads) pack_weight_f16x2_kernel(const P
     const long o = 32L * block + m;
     const int pieces = I >> 3;                            // per row; thread t takes pieces t / 32, + 32, ...
     const long total = (long)O_pad * I;
-    if (tid < 32) row_max[tid] = 0;
+    if (tid < 32) row_max[tid] = row_odd[tid] = 0;
     __syncthreads();
     const float* row = W + (o < O ? o : 0) * so;
     auto load = [&](float (&v)[8], int piece) {
@@ -97,26 +104,37 @@ __global__ void __launch_bounds__(kPackThreads) pack_weight_f16x2_kernel(const P
     };
     float keep[kPackRegs][8];
     unsigned mx = 0;
+    bool odd = false;
+    auto largest = [&](float v) {
+        const unsigned b = __float_as_uint(fabsf(v));
+        if (b >= 0x7f800000u) odd = true;
+        else mx = b > mx ? b : mx;
+    };
 #pragma unroll
     for (int u = 0; u < kPackRegs; u++) {
         const int piece = (tid >> 5) + 32 * u;
         if (piece < pieces) {
             load(keep[u], piece);
 #pragma unroll
-            for (int j = 0; j < 8; j++) { const unsigned b = __float_as_uint(fabsf(keep[u][j])); mx = b > mx ? b : mx; }
+            for (int j = 0; j < 8; j++) largest(keep[u][j]);
         }
     }
     for (int piece = (tid >> 5) + 32 * kPackRegs; piece < pieces; piece += 32) {
         float v[8];
         load(v, piece);
 #pragma unroll
-        for (int j = 0; j < 8; j++) { const unsigned b = __float_as_uint(fabsf(v[j])); mx = b > mx ? b : mx; }
+        for (int j = 0; j < 8; j++) largest(v[j]);
     }
     atomicMax(&row_max[m], mx);
+    if (odd) row_odd[m] = 1;
     __syncthreads();
     float inv;
     const float s = pow2_scale(__uint_as_float(row_max[m]), &inv);
-    if (tid < 32) inv_scale[o] = inv;
+    if (tid < 32) {
+        inv_scale[o] = row_odd[m] ? mark_weight(inv) : inv;
+        const int marked = __any(row_odd[m]);
+        if (tid == 0) marked_blocks(inv_scale, O_pad)[block] = marked;
+    }
     auto store = [&](const float (&v)[8], int piece) {
         halfx8 hi, lo;
 #pragma unroll
@@ -194,8 +212,11 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// (waves per SIMD that the registers of the narrow tiles are held to: the epilogue's rare paths would cost one otherwise)
+constexpr int streaming_waves(int waves, int ni) { return waves == 4 && ni <= 2 ? 6 - ni : 1; }
+
 template <int WAVES, int NI>
-__global__ void __launch_bounds__(64 * WAVES)
+__global__ void __launch_bounds__(64 * WAVES, streaming_waves(WAVES, NI))
 linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restrict__ w_inv, const float* __restrict__ X,
                          const float* __restrict__ xmax, int xmax_parts, long xmax_stride, long xmax_div, long R, int I,
                          int O, int O_pad, const float* __restrict__ bias, int act, int accumulate,
@@ -236,6 +257,7 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
     const long ld_row = my_row < R ? my_row : R - 1;
     const float* xrow = X + ld_row * I + 16 * g;
     float sx;
+    bool odd_cols, odd;                                      // this wave has columns, or anything, that the pieces cannot carry
     {
         float amax = 0.f;
         const float* xm = xmax + (ld_row / xmax_div) * xmax_stride;
@@ -243,7 +265,14 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
         amax = fmaf(amax, bound_mul, bound_add);             // the caller's bound of |x| is bound_mul * xmax + bound_add
         float inv;
         sx = pow2_scale(amax, &inv);
-        if (g == 0) inv_sx[wave * 32 + m] = inv;
+        if (g == 0) inv_sx[wave * 32 + m] = beyond_split(amax) ? __builtin_nanf("") : inv;
+        const int* marked = marked_blocks(w_inv, O_pad) + n0 / 32;
+        int any = 0;
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++) any |= marked[ni];   // (scalar loads)
+        asm volatile("" : "+s"(any));                        // (here, where others are waited for anyway, not in the epilogue)
+        odd_cols = any != 0;
+        odd = odd_cols || __any(beyond_split(amax));
     }
     const _Float16* wsrc[kPer];
     int wdst[kPer];
@@ -329,7 +358,13 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
         __syncthreads();
     }
 
-    const bool full_cols = n0 + TN <= O;
+    if constexpr (kRuns)
+        if (out_T == 9) {                                    // (epilogue_runs has barriers: all waves go the same way)
+            bool row = false;
+            for (int r = lane; r < TM; r += 64) { const float isx = inv_sx[r]; row |= isx != isx; }
+            odd |= __any(row);
+        }
+    const bool full_cols = n0 + TN <= O && !odd;
     // ---- fast path, plain rows: y (rows, O)
     auto epilogue_rows = [&](auto act_tag, auto acc_tag, auto some_tag) {
         constexpr int kAct = decltype(act_tag)::value;
@@ -442,7 +477,7 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
         return;
     }
 
-    // ---- general path: partial column tiles, or components with bias / activation
+    // ---- general path: partial column tiles, components with bias / activation, rows or columns beyond the pieces
     float rmax[16];
 #pragma unroll
     for (int q = 0; q < 16; q++) rmax[q] = 0.f;
@@ -456,20 +491,35 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
         for (int q = 0; q < 16; q++) {
             const int rl = wave * 32 + 8 * (q / 4) + 4 * g + (q % 4);
             const long r = r0 + rl;
-            if (r < R) {
+            const float isx = inv_sx[rl];
+            if (r < R && isx == isx && iw == iw) {
                 const long row = r / out_T;
                 const long addr = (row * O + n) * out_T + (r - row * out_T);
-                float v = activate(acc[ni][q] * inv_sx[rl] * iw + (r < bias_rows ? bv : 0.f), act);
+                float v = activate(acc[ni][q] * isx * iw + (r < bias_rows ? bv : 0.f), act);
                 if (accumulate) v += Y[addr];
                 Y[addr] = v;
                 rmax[q] = fmaxf(rmax[q], fabsf(v));
             }
         }
     }
+    if (odd) {
+#pragma unroll 1
+        for (int k = 0; k < 16 * NI; k++) {
+            const int n = n0 + (k >> 4) * 32 + m, q = k & 15, rl = wave * 32 + 8 * (q / 4) + 4 * g + (q % 4);
+            const long r = r0 + rl;
+            if (n >= O || r >= R) continue;
+            const float isx = inv_sx[rl], iw = w_inv[n];
+            if (isx == isx && iw == iw) continue;
+            const long row = r / out_T, addr = (row * O + n) * out_T + (r - row * out_T);
+            const float v = activate(row_in_fp32(X + r * I, Wp, plane_elems, n, I, iw) + (bias && r < bias_rows ? bias[n] : 0.f), act);
+            Y[addr] = accumulate ? v + Y[addr] : v;
+        }
+    }
     if (ymax) {
 #pragma unroll
         for (int q = 0; q < 16; q++) {
-            float mx = rmax[q];
+            const float isx = inv_sx[wave * 32 + 8 * (q / 4) + 4 * g + (q % 4)];
+            float mx = odd_cols || isx != isx ? __builtin_inff() : rmax[q];        // (no bound: the next layer takes the row in fp32)
 #pragma unroll
             for (int d = 1; d < 32; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
             const long r = r0 + wave * 32 + 8 * (q / 4) + 4 * g + (q % 4);
@@ -517,7 +567,7 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
         amax = fmaf(amax, bound_mul, bound_add);
         float inv;
         sx = pow2_scale(amax, &inv);
-        if (wave == 0 && g == 0) inv_sx[m] = inv;
+        if (wave == 0 && g == 0) inv_sx[m] = beyond_split(amax) ? __builtin_nanf("") : inv;
     }
     // lane's fragment of W for MFMA step s, column block ni: row n0 + 32 ni + m, k = k0 + 16 g + 8 s .. + 8
     const _Float16* wrow = Wp + packed_piece(n0, lane, I);
@@ -582,6 +632,7 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
     // row are neighbours, so its maximum is a shuffle away)
     constexpr int kPer = 32 * TN / THREADS;
     static_assert(32 * TN % THREADS == 0 && THREADS % TN == 0 && TN <= 64, "whole rows per pass, a row within a wave");
+    bool odd = false;                                         // an element of a row or column that the pieces cannot carry
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
         const int e = tid + THREADS * j;
@@ -595,15 +646,34 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
         if (r < R && n < O) {
             const long row = r / out_T;
             const long addr = (row * O + n) * out_T + (r - row * out_T);
-            v = activate(sum * inv_sx[rl] * w_inv[n] + (bias && r < bias_rows ? bias[n] : 0.f), act);
-            if (accumulate) v += Y[addr];
-            Y[addr] = v;
+            const float isx = inv_sx[rl], iw = w_inv[n], bv = bias && r < bias_rows ? bias[n] : 0.f;
+            if (isx == isx && iw == iw) {
+                v = activate(sum * isx * iw + bv, act);
+                if (accumulate) v += Y[addr];
+                Y[addr] = v;
+            } else {
+                odd = true;
+                v = __builtin_inff();                         // (no bound: the next layer takes the row in fp32)
+            }
         }
         if (ymax) {
             float mx = fabsf(v);
 #pragma unroll
             for (int d = 1; d < TN; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
             if (col == 0 && r < R) ymax[r * tiles_n + tile_n] = mx;
+        }
+    }
+    if (odd) {
+#pragma unroll 1
+        for (int j = 0; j < kPer; j++) {
+            const int e = tid + THREADS * j, rl = e / TN, n = n0 + e - rl * TN;
+            const long r = r0 + rl;
+            if (r >= R || n >= O) continue;
+            const float isx = inv_sx[rl], iw = w_inv[n];
+            if (isx == isx && iw == iw) continue;
+            const long row = r / out_T, addr = (row * O + n) * out_T + (r - row * out_T);
+            const float v = activate(row_in_fp32(X + r * I, Wp, plane_elems, n, I, iw) + (bias && r < bias_rows ? bias[n] : 0.f), act);
+            Y[addr] = accumulate ? v + Y[addr] : v;
         }
     }
 }
@@ -688,7 +758,7 @@ extern "C" {
 int mg_linear_f16x2_packed_weight_bytes(int dim_in, int dim_out, size_t* bytes) {
     MG_REQUIRE(bytes != nullptr && dim_in >= 0 && dim_out >= 0, "mg_linear_f16x2_packed_weight_bytes: bad argument");
     const size_t o_pad = (size_t)o_pad_of(dim_out);
-    *bytes = 2 * o_pad * (size_t)dim_in * sizeof(_Float16) + o_pad * sizeof(float);
+    *bytes = 2 * o_pad * (size_t)dim_in * sizeof(_Float16) + o_pad * sizeof(float) + o_pad / 32 * sizeof(int);
     return MG_OK;
 }
 

@@ -649,3 +649,74 @@ def test_linear_few_inputs(ops, inds, dim_in, rows, dim_out):
     else:
         y2 = ops.tensor_linear_fwd(inds, W.cuda(), x.cuda(), y_layout=ops.LAYOUT_COMP_CHAN)
         assert torch.equal(y2.reshape(rows, T, dim_out).transpose(1, 2), y.reshape(rows, dim_out, T))
+
+
+# few rows (the split reduction: one, two column blocks, four and eight waves), many (row streaming, with a partial column
+# tile, with the epilogue in runs of nine components)
+@pytest.mark.parametrize("inds,rows,dim_in,dim_out", [(0, 1, 64, 8), (0, 40, 128, 512), (0, 200, 1280, 16), (0, 255, 256, 256),
+                                                      (0, 9000, 64, 300), (0, 9000, 128, 256), (1, 330, 128, 384),
+                                                      (1, 9000, 64, 192), (2, 120, 64, 64), (2, 3001, 64, 256)])
+def test_rows_and_columns_the_fp16_pieces_cannot_carry(ops, inds, rows, dim_in, dim_out):
+    """Infinite and very large entries of x, and infinite weights, through the split-fp16 kernels: infinities and NaN where
+    float64 arithmetic has them, finite results to the tolerance of a sum in fp32, other rows and columns bit for bit as without them.
+    Then the same with bias, activation and accumulation, and through the row maxima into a second layer."""
+    assert ops.get_linear_mode() == ops.LINEAR_F16X2
+    g = torch.Generator().manual_seed(rows + dim_in)
+    T = 3 ** inds
+    x = torch.randn(rows, dim_in, *([3] * inds), generator=g)
+    W = torch.randn(dim_out, dim_in, generator=g) / dim_in ** 0.5
+    W[dim_out // 3] = torch.randint(1, 5, (dim_in,), generator=g).float() / 4     # (its low pieces are zeros)
+    W[dim_out // 2, 1] = 0.0
+    inf = float("inf")
+    odd = sorted({0, rows // 2, rows - 1})
+    bad = x.clone().reshape(rows, dim_in, T)
+    bad[odd[0], 1, 0] = inf
+    bad[odd[-1], dim_in - 1, T - 1] = -inf
+    bad[odd[len(odd) // 2], :, T // 2] *= 1e30                                    # (one component only: a row of its own)
+    bad = bad.reshape(x.shape)
+
+    def close(y, want, what):
+        y, want = y.cpu().double(), want.cpu()
+        assert torch.equal(torch.isnan(y), torch.isnan(want)), what
+        assert torch.equal(torch.where(torch.isinf(y), y, 0.0), torch.where(torch.isinf(want), want, 0.0)), what
+        y, want = (torch.where(torch.isfinite(t), t, 0.0).reshape(rows, -1, T) for t in (y, want))
+        scale = want.abs().amax(1, keepdim=True).clamp_min(1e-30)
+        assert float(((y - want).abs() / scale).max()) <= dim_in * 2 ** -23, what       # the chain's bound, K roundings of half an ulp, twice
+
+    def product(x_, W_):
+        return OP.tensor_linear(inds, W_.double(), x_.double())
+
+    plain = ops.tensor_linear_fwd(inds, W.cuda(), x.cuda())
+    y = ops.tensor_linear_fwd(inds, W.cuda(), bad.cuda())
+    close(y, product(bad, W), "infinite entries")
+    same = (bad == x).reshape(rows, dim_in, T).all(1)                                    # (rows, components) left as they were
+    keep = same[:, None].expand(rows, dim_out, T)
+    assert torch.equal(y.cpu().reshape(rows, dim_out, T)[keep], plain.cpu().reshape(rows, dim_out, T)[keep])
+    Wi = W.clone()
+    Wi[dim_out - 1, 0], Wi[1, dim_in - 1] = inf, -inf
+    yw = ops.tensor_linear_fwd(inds, Wi.cuda(), x.cuda())
+    close(yw, product(x, Wi), "infinite weights")
+    cols = [o for o in range(dim_out) if o not in (1, dim_out - 1)]
+    assert torch.equal(yw.cpu().reshape(rows, dim_out, T)[:, cols], plain.cpu().reshape(rows, dim_out, T)[:, cols])
+    if inds > 0:
+        base = torch.randn(y.shape, generator=g)
+        rows_ = ops.components_as_rows(inds, bad.cuda())
+        out = ops.tensor_linear_f16x2(W.cuda(), rows_[0][:, :dim_in].contiguous(), rows_[1], out=base.cuda(), accumulate=True, out_comps=T)
+        assert torch.equal(torch.nan_to_num(out), torch.nan_to_num(y + base.cuda()))
+        return
+    b = torch.randn(dim_out, generator=g)
+    base = torch.randn(rows, dim_out, generator=g)
+    z = product(bad, W) + b.double()
+    for act, f in ((ops.ACT_NONE, lambda t: t), (ops.ACT_LEAKY, lambda t: torch.nn.functional.leaky_relu(t, 0.1))):
+        out = ops.tensor_linear_fwd(0, W.cuda(), bad.cuda(), bias=b.cuda(), act=act, out=base.cuda(), accumulate=True)
+        close(out, f(z) + base.double(), "bias, activation, accumulated")
+    h, hmax = ops.tensor_linear_f16x2(W.cuda(), bad.cuda(), ops.row_absmax(bad.cuda()), bias=b.cuda(), want_rowmax=True)
+    assert bool((hmax.amax(1) >= torch.nan_to_num(h, nan=0.0, posinf=inf, neginf=-inf).abs().amax(1)).all())
+    if dim_out % 32 == 0 and dim_out >= 64:
+        W2 = torch.randn(64, dim_out, generator=g) / dim_out ** 0.5
+        y2 = ops.tensor_linear_f16x2(W2.cuda(), h, hmax)
+        want = h.cpu().double() @ W2.double().T
+        finite = torch.isfinite(want).all(1)
+        assert torch.equal(torch.isfinite(y2.cpu()).all(1), finite)
+        err = (y2.cpu().double() - want)[finite].abs() / want[finite].abs().amax(1, keepdim=True)
+        assert float(err.max()) <= dim_out * 2 ** -23
