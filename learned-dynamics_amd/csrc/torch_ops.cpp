@@ -235,9 +235,20 @@ std::pair<at::Tensor, at::Tensor> components_to_rows(const at::Tensor& x, int64_
 
 bool power_of_two(int64_t v) { return v > 0 && (v & (v - 1)) == 0; }
 
-// rows x components from which a tensor linear goes through plain component rows and the split-fp16 kernels; in sequential
-// order the old crossover stays: an element's order of summation must not change with the number of rows in between
-constexpr int64_t kComponentRows = 960, kComponentRowsSequential = 32768;
+// Whether a tensor linear of R = rows x components goes through plain component rows and the split-fp16 kernels.
+// Channels: from 32 its error against float64 is no larger than that of fp32 products summed in k order (2-norm, 32 channels
+// 0.95e-7 against 1.03e-7, 64 1.0e-7 against 1.45e-7, 128 1.0e-7 against 2.0e-7); with fewer the rounding of the pieces outweighs
+// the shorter sum (16 channels 0.88e-7 against 0.74e-7, 24 0.91e-7 against 0.89e-7), and they stay in fp32 below 32 768.
+// R: the generic kernel is the slower one at every R that was measured, with the transposition counted (64 -> 64: 17.3 against
+// 7.1 us at 960, 18.0 against 12.1 at 15 360; 256 -> 256: 32.5 against 8.9 and 47 against 30; three components), down to 96 (16.8
+// against 6.8).  The line at 960 is no crossover: calls below it have kept fp32 arithmetic in k order.
+// With `sequential` the line is 32 768 for every width: below it an element's order of summation does not depend on R.
+constexpr int64_t kComponentRows = 960, kComponentRowsF32 = 32768, kComponentChannels = 32;
+bool component_rows_take(int64_t R, int64_t dim_in, int64_t dim_out, bool sequential) {
+    if (dim_out < 64) return false;
+    if (sequential) return R >= kComponentRowsF32;
+    return dim_in > 8 && R >= (dim_in >= kComponentChannels ? kComponentRows : kComponentRowsF32);
+}
 
 std::tuple<at::Tensor, OptTensor> linear_fwd(int64_t inds, const at::Tensor& W, const at::Tensor& x, const OptTensor& bias,
                                              int act, const OptTensor& out, bool accumulate, int x_layout, int y_layout,
@@ -299,12 +310,12 @@ std::tuple<at::Tensor, OptTensor> linear_fwd(int64_t inds, const at::Tensor& W, 
         return emit ? &ymax : nullptr;
     };
     const int64_t k_pad = (dim_in + 31) / 32 * 32;
-    if (mode == kModeF16x2 && inds > 0 && x_layout == 0 && R >= (sequential ? kComponentRowsSequential : kComponentRows) &&
-        (sequential || dim_in > 8) && dim_out >= 64 && !row_bound.has_value() &&
+    if (mode == kModeF16x2 && inds > 0 && x_layout == 0 && component_rows_take(R, dim_in, dim_out, sequential) &&
+        !row_bound.has_value() &&
         (y_layout == 1 || !(want_rowmax || accumulate || bias.has_value() || act != kActNone))) {
         // (row, chan, comp) -> (row, comp, chan) rows, then the plain-row matrix path: its component-major output is
         // written at the full store rate, and with the reference's output layout its component epilogue still beats the
-        // generic kernel (61 against 104 us for 16384 x 128 x 3 -> 384, 9 against 22 us for 337 x 128 x 3 -> 384)
+        // generic kernel (61 against 104 us for 16384 x 128 x 3 -> 384)
         at::Tensor x2, x2max;
         if (x2_given.has_value() && x2_given->dim() == 2 && x2_given->size(0) == R && x2_given->size(1) == k_pad) {
             x2 = *x2_given;
@@ -1112,6 +1123,7 @@ void register_ops(pybind11::module_& m) {
     m.def("row_absmax", &row_absmax);
     m.def("linear_f16x2", &linear_f16x2);
     m.def("linear_fwd", &linear_fwd);
+    m.def("component_rows_take", &component_rows_take);
     m.def("linear_wgrad", &linear_wgrad);
     m.def("silu_order", &silu_order);
     m.def("linear_chain", &linear_chain);

@@ -1138,9 +1138,6 @@ def tensor_linear_f16x2(W, x, x_rowmax=None, bias=None, act=ACT_NONE, out=None, 
 
 
 LAYOUT_CHAN_COMP, LAYOUT_COMP_CHAN = 0, 1
-# rows x components from which a tensor linear goes through plain component rows and the split-fp16 kernels
-# (kComponentRows of csrc/torch_ops.cpp)
-COMPONENT_ROWS_MIN = 960
 
 
 def components_as_rows(inds, x):
@@ -1155,7 +1152,7 @@ def components_as_rows(inds, x):
     dim_in = int(x.size(x.dim() - 1 - inds))
     rows = x.numel() // (dim_in * T) if dim_in else 0
     k_pad = (dim_in + 31) // 32 * 32
-    if (get_linear_mode() != LINEAR_F16X2 or rows * T < COMPONENT_ROWS_MIN or dim_in <= 8 or k_pad > 256
+    if (get_linear_mode() != LINEAR_F16X2 or not _ext.component_rows_take(rows * T, dim_in, 64, False) or k_pad > 256
             or k_pad & (k_pad - 1)):
         return None
     with _on(x.device):

@@ -634,7 +634,7 @@ def test_linear_f16x2_split_reduction(ops, rows, dim_in, dim_out, act):
         assert torch.equal(a, ops.tensor_linear_fwd(0, W, many, bias=b, act=act)[:rows])
 
 
-@pytest.mark.parametrize("inds,dim_in", [(0, 1), (0, 8), (0, 20), (0, 32), (1, 1), (1, 8), (2, 3)])
+@pytest.mark.parametrize("inds,dim_in", [(0, 1), (0, 8), (0, 20), (0, 32), (1, 1), (1, 8), (2, 3), (1, 9), (1, 16), (2, 13), (2, 16)])
 @pytest.mark.parametrize("rows,dim_out", [(1, 5), (63, 256), (700, 300)])
 def test_linear_few_inputs(ops, inds, dim_in, rows, dim_out):
     g = torch.Generator().manual_seed(rows + dim_in)
@@ -720,3 +720,23 @@ def test_rows_and_columns_the_fp16_pieces_cannot_carry(ops, inds, rows, dim_in, 
         assert torch.equal(torch.isfinite(y2.cpu()).all(1), finite)
         err = (y2.cpu().double() - want)[finite].abs() / want[finite].abs().amax(1, keepdim=True)
         assert float(err.max()) <= dim_out * 2 ** -23
+
+
+@pytest.mark.parametrize("inds,rows,dim_in,dim_out", [(1, 2048, 16, 64), (2, 2048, 16, 256), (2, 1000, 24, 64), (1, 1000, 32, 64),
+                                                      (2, 500, 64, 64), (1, 337, 128, 384), (0, 1, 64, 256), (0, 200, 64, 8),
+                                                      (0, 100, 256, 768), (0, 18432, 1280, 16)])
+def test_small_problems_are_no_less_precise_than_fp32(ops, inds, rows, dim_in, dim_out):
+    """Whatever kernel these sizes take by default is as close to float64 as products and sums in fp32 are (2-norms)."""
+    g = torch.Generator().manual_seed(rows + dim_in)
+    x = torch.randn(rows, dim_in, *([3] * inds), generator=g)
+    x = x * torch.exp(0.5 * torch.randn(rows, dim_in, *([1] * inds), generator=g))
+    W = torch.randn(dim_out, dim_in, generator=g) / dim_in ** 0.5
+    ref = OP.tensor_linear(inds, W.double(), x.double())
+    err = lambda: float((ops.tensor_linear_fwd(inds, W.cuda(), x.cuda()).cpu().double() - ref).norm() / ref.norm())
+    default = err()
+    ops.set_linear_mode(ops.LINEAR_FP32_MFMA)
+    try:
+        fp32 = err()
+    finally:
+        ops.set_linear_mode(ops.LINEAR_F16X2)
+    assert default <= 1.01 * fp32, (default, fp32)               # (where both run the same kernel they are equal)
