@@ -17,11 +17,12 @@ import math
 import torch
 import torch.autograd.forward_ad as fwAD
 import torch.nn.functional as F
+import torch.nn.modules.module as _nn_module
 
 from . import graph_layers as gl
 from . import ops
 from .codegen_tensor_products import Bee
-from .tensor_products import tensor_linear
+from .tensor_products import TensLinear, tensor_linear
 
 
 def has_tangent(t):
@@ -46,6 +47,16 @@ def wants_grad(module, *tensors):
     if any(t is not None and t.requires_grad for t in tensors):
         return True
     return any(p.requires_grad for p in module.parameters())
+
+
+def plain_call(module, cls):
+    """True when calling the module runs cls.forward and nothing else: not a subclass or another module in its place, no
+    hooks, no compiled call.  What the fused functions, which read a submodule's parameters and enqueue, may stand for."""
+    own = module.__dict__
+    return (type(module) is cls and "forward" not in own and own.get("_compiled_call_impl") is None
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                     or _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks
+                     or _nn_module._global_backward_hooks or _nn_module._global_backward_pre_hooks))
 
 
 def _one_sided(a, b):
@@ -265,7 +276,7 @@ def _fused(params, *tensors):
     """Whether the fused functions take these: float32 on the device, rows of whole 16-byte pieces, no tangents on the
     parameters."""
     return (all(t is None or (t.is_cuda and t.dtype == torch.float32 and t.data_ptr() % 16 == 0 and t.numel() > 0) for t in tensors)
-            and all(p.is_cuda and p.dtype == torch.float32 and p.is_contiguous() and p.shape[0] % 4 == 0 for p in params)
+            and all(p is not None and p.is_cuda and p.dtype == torch.float32 and p.is_contiguous() and p.shape[0] % 4 == 0 for p in params)
             and not any(has_tangent(p) for p in params))
 
 
@@ -849,22 +860,27 @@ class _PainnUpdate(torch.autograd.Function):
         return (None,) + tuple(g if nd else None for g, nd in zip(grads, need[1:]))
 
 
-def _update_pieces(upd, params, x_a, x_v):
-    """painn.Update out of differentiable pieces"""
+def _update_pieces(upd, params, x_a, x_v, maps=None):
+    """painn.Update out of differentiable pieces; params: gamma, beta and the MLP's behind the three maps' weights, which
+    `maps` (callables) stand in for."""
     n = upd.n
-    W_l, W_r, W_v = params[:3]
     x_v = x_v.contiguous()
-    v_l, v_r = (tensor_linear(1, W, x_v) for W in (W_l, W_r))
+    lin_l, lin_r, lin_v = maps or [lambda x, W=W: tensor_linear(1, W, x) for W in params[:3]]
+    v_l, v_r = lin_l(x_v), lin_r(x_v)
     ip = (v_l * v_r).sum(-1)
-    y = _mlp_rows(params[5:], torch.cat([x_a, torch.linalg.vector_norm(v_r, dim=-1)], dim=-1))
-    v = tensor_linear(1, W_v, x_v) * y[..., :n, None]
-    a = scal_group_norm(upd.gn, ip * y[..., n:2 * n], params[3], params[4]) + y[..., 2 * n:]
+    y = _mlp_rows(params[-6:], torch.cat([x_a, torch.linalg.vector_norm(v_r, dim=-1)], dim=-1))
+    v = lin_v(x_v) * y[..., :n, None]
+    a = scal_group_norm(upd.gn, ip * y[..., n:2 * n], params[-8], params[-7]) + y[..., 2 * n:]
     return a, v / torch.sqrt(add((v ** 2).sum(-1, keepdim=True), 1.))
 
 
 def painn_update(upd, x_a, x_v):
     """archs/meanflow_painn8.py:63-75"""
-    params = [upd.lin_l.W, upd.lin_r.W, upd.lin_v.W, upd.gn.gamma, upd.gn.beta, *_mlp_parameters(upd.mlp)]
+    maps = (upd.lin_l, upd.lin_r, upd.lin_v)
+    params = [upd.gn.gamma, upd.gn.beta, *_mlp_parameters(upd.mlp)]
+    if not all(plain_call(lin, TensLinear) for lin in maps):
+        return _update_pieces(upd, params, x_a, x_v, maps)
+    params = [lin.W for lin in maps] + params
     pairs = [tuple(_dense(t) for t in _unpack(x)) for x in (x_a, x_v)]
     (a, a_t), (v, v_t) = pairs
     if a_t is not None and v_t is None:

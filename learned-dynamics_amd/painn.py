@@ -65,11 +65,17 @@ def _linear(x, lin, act, bound=None, want_bound=True):
 _MLP_ACTS = (ops.ACT_SILU, ops.ACT_SILU, ops.ACT_NONE)
 
 
-def _mlp_params(mlp, last=None):
-    """([weights], [biases]) of an MLP's three linears; last: a layer to use in the last one's place."""
-    m = mlp.layers._modules
-    lins = (m["0"], m["2"], last if last is not None else m["4"])
-    return [lin.weight for lin in lins], [lin.bias for lin in lins]
+def _mlp_params(mlp):
+    """([weights], [biases]) of an MLP's three linears, or None when one has no bias: the calls that take these lists want all
+    of them."""
+    lins = list(mlp.layers._modules.values())[0:5:2]
+    biases = [lin.bias for lin in lins]
+    return None if any(b is None for b in biases) else ([lin.weight for lin in lins], biases)
+
+
+def _plain_params(mlp):
+    """_mlp_params of a submodule whose call may be replaced by one that reads its parameters, else None."""
+    return _mlp_params(mlp) if diff.plain_call(mlp, MLP) else None
 
 
 class MLP(nn.Module):
@@ -92,7 +98,11 @@ class MLP(nn.Module):
         if diff.wants_grad(self, x_a):
             return diff.mlp_silu(self, x_a)
         h = x_a.reshape(-1, x_a.shape[-1]).contiguous()
-        y = ops.linear_chain(h, *_mlp_params(self), _MLP_ACTS, bound)
+        params = _mlp_params(self)
+        if params is not None:
+            y = ops.linear_chain(h, *params, _MLP_ACTS, bound)
+        else:
+            y = self.after_first(*_linear(h, self.layers[0], ops.ACT_SILU, bound))
         return y if x_a.dim() == 2 else y.reshape(*x_a.shape[:-1], -1)
 
     def hidden(self, x, bound=None):
@@ -152,8 +162,20 @@ class Update(nn.Module):
         if cache.get("stamp") != stamp:                                         # (3n, n): one GEMM for l, r, v; kept
             with ops.derived_tensors():                                         # while the weights are unchanged, so
                 cache.update(stamp=stamp, W=torch.cat(params, dim=0))           # its packed planes stay valid too
-        W = cache["W"]
-        return ops.painn_update(x_a.contiguous(), x_v.contiguous(), W, *_mlp_params(self.mlp), self.gn, residual)
+        W, mlp = cache["W"], _plain_params(self.mlp)
+        x_a, x_v = x_a.contiguous(), x_v.contiguous()
+        if mlp is not None and diff.plain_call(self.gn, ScalGroupNorm):
+            return ops.painn_update(x_a, x_v, W, *mlp, self.gn, residual)
+        # with the submodules called as such (hooks, something else in their place)
+        B, N, n = x_a.shape
+        flat_a, flat_v = x_a.reshape(B * N, n), x_v.reshape(B * N, n, 3)
+        lrv = ops.tensor_linear_fwd(1, W, flat_v, y_layout=ops.LAYOUT_COMP_CHAN)
+        ip, cat, cat_max = ops.painn_update_pre(lrv, flat_a, want_rowmax=True)
+        y = self.mlp(cat, cat_max)
+        y3 = y.reshape(B, N, 3 * n)
+        out_a = self.gn(ip.reshape(B, N, n), mul=y3[..., n:2 * n], add=y3[..., 2 * n:], res=x_a if residual else None)
+        out_v = ops.painn_update_vec(lrv, y, flat_v if residual else None)
+        return out_a, out_v.reshape(B, N, n, 3)
 
 
 class Message(nn.Module):
@@ -182,6 +204,8 @@ class Message(nn.Module):
 
     def filters(self, r_ij):
         """(edges, 3) -> (edges, 4n): the per-edge filter, the one large per-edge tensor."""
+        if _plain_params(self.mlp_dist) is None:
+            return self.mlp_dist(ops.painn_radial_encode(r_ij, self.n_rbf, self.r0), ops.linear_in_unit_bound(r_ij.device))
         return self.mlp_dist.after_first(*self._hidden(r_ij))
 
     use_sliced = True
@@ -263,15 +287,17 @@ class Message(nn.Module):
         return kept[1]
 
     def _evaluate_filter_table(self, rows, shift=0.0):
-        if diff.wants_grad(self.mlp_dist):
-            return self.mlp_dist(self._grid_encoding(rows, shift, self.mlp_dist.layers[0].weight.device))
-        return ops.filter_grid(*self._grid_inputs(rows, shift))
+        params = _plain_params(self.mlp_dist)
+        if params is None or diff.wants_grad(self.mlp_dist):
+            device = self.mlp_dist.layers[0].weight.device
+            return self.mlp_dist(self._grid_encoding(rows, shift, device), ops.linear_in_unit_bound(device))
+        return ops.filter_grid(*self._grid_inputs(params, rows, shift))
 
-    def _grid_inputs(self, rows, shift=0.0):
-        """(encodings of the grid, a unit bound of them, weights, biases) for ops.filter_grid.  A reduction dimension of n_rbf below
-        GRID_K is less than what the matrix path takes: the encodings (constants of the grid) and the weight's columns
-        are then padded with zeros, which leaves every product as it was."""
-        W, b = _mlp_params(self.mlp_dist)
+    def _grid_inputs(self, params, rows, shift=0.0):
+        """(encodings of the grid, a unit bound of them, weights, biases) for ops.filter_grid, params: mlp_dist's.  A reduction
+        dimension of n_rbf below GRID_K is less than what the matrix path takes: the encodings (constants of the grid) and the
+        weight's columns are then padded with zeros, which leaves every product as it was."""
+        W, b = params
         device = W[0].device
         pad = self.n_rbf < self.GRID_K and ops.get_linear_mode() == ops.LINEAR_F16X2 and W[0].shape[0] >= 8
         return (self._grid_encoding(rows, shift, device, self.GRID_K if pad else None), ops.linear_in_unit_bound(device), W, b)
@@ -293,9 +319,10 @@ class Message(nn.Module):
         if key not in cache:
             cache[key] = self._grid_phases(rows, shift).to(device).contiguous()
         with ops.derived_tensors():
-            h = ops.linear_f64(L[0].weight.detach(), L[0].bias.detach(), cache[key], ops.ACT_SILU)
-            h = ops.linear_f64(L[2].weight.detach(), L[2].bias.detach(), h, ops.ACT_SILU)
-            return ops.linear_f64(L[4].weight.detach(), L[4].bias.detach(), h, ops.ACT_NONE)
+            h = cache[key]
+            for lin, act in zip(list(L)[0:5:2], _MLP_ACTS):
+                h = ops.linear_f64(lin.weight.detach(), None if lin.bias is None else lin.bias.detach(), h, act)
+            return h
 
     def table_error(self, rows):
         """max over the grid's midpoints and the 4n filter columns of
@@ -339,29 +366,43 @@ class Message(nn.Module):
         B, N, n = x_a.shape
         x_a, x_v, r_ij = x_a.contiguous(), x_v.contiguous(), r_ij.contiguous()
         E = r_ij.shape[0]
-        if self.use_table and n % 4 == 0 and E >= 4 * self.TABLE_ROWS[0]:
+        actv_mlp, dist_mlp = _plain_params(self.mlp_actv), _plain_params(self.mlp_dist)
+        plain = actv_mlp is not None and dist_mlp is not None
+        flat_a, flat_v = x_a.reshape(B * N, n), x_v.reshape(B * N, n, 3)
+        res_a, res_v = (flat_a, flat_v) if residual else (None, None)
+        if self.use_table and isinstance(self.mlp_dist, MLP) and n % 4 == 0 and E >= 4 * self.TABLE_ROWS[0]:
             rows = self.table_rows()
             sliced = rows and rows <= ops.PAINN_SLICED_MAX_ROWS and n % ops.PAINN_SLICE == 0 and self.use_sliced
+            if (sliced or (rows and E >= 4 * rows)) and not plain:
+                # (the submodules called as such: hooks, something else in their place)
+                out_a, out_v = ops.painn_table_message(graph.row_ptr, graph.dst32, r_ij, self.filter_table(rows), 2.0 * self.r0,
+                                                       self.mlp_actv(flat_a), flat_v, self.epsilon, res_a, res_v)
+                return out_a.reshape(B, N, n), out_v.reshape(B, N, n, 3)
             if sliced or (rows and E >= 4 * rows):
                 # The grid is re-evaluated in every call (a few thousand rows): nothing of a forward is cached.  Where it
                 # fits in LDS, actv comes out of its MLP with the columns regrouped slice by slice, and the rows are taken
                 # in cell order when the graph has one: consecutive rows then gather the same neighbours.
                 order = getattr(graph, "cell_order", None) if sliced and self.use_cell_order else None
                 table = self.filter_table(rows) if self.keep_table else None
-                return ops.painn_message_grid(graph.row_ptr, graph.dst32, r_ij, order, x_a, x_v,
-                                              *_mlp_params(self.mlp_actv, self._sliced_actv_last() if sliced else None),
-                                              *self._grid_inputs(rows), table, 2.0 * self.r0, self.epsilon, sliced, residual)
+                if sliced:
+                    last, (W, b) = self._sliced_actv_last(), actv_mlp
+                    actv_mlp = [*W[:2], last.weight], [*b[:2], last.bias]
+                return ops.painn_message_grid(graph.row_ptr, graph.dst32, r_ij, order, x_a, x_v, *actv_mlp,
+                                              *self._grid_inputs(dist_mlp, rows), table, 2.0 * self.r0, self.epsilon, sliced, residual)
         if getattr(graph, "padded", False):
             # the edge arrays are longer than the graph: only the kernels above, which reach the edges through
             # row_ptr, are valid; the per-edge GEMMs below would also process the rows past the edge count
             raise RuntimeError("Message.forward on a capacity-sized graph needs the filter-grid path "
                                "(n a multiple of 16, a grid accepted for these weights, edge capacity >= 4 x grid rows)")
-        if E < self.FOLD_EDGES or not ops.painn_filter_message_supported(n, 4 * n, E):
-            return ops.painn_message_edges(graph.row_ptr, graph.dst32, r_ij, x_a, x_v, *_mlp_params(self.mlp_actv),
-                                           *_mlp_params(self.mlp_dist), self.r0, self.epsilon, residual)
-        flat_a, flat_v = x_a.reshape(B * N, n), x_v.reshape(B * N, n, 3)
-        res_a, res_v = (flat_a, flat_v) if residual else (None, None)
+        fold = E >= self.FOLD_EDGES and ops.painn_filter_message_supported(n, 4 * n, E)
+        if plain and not fold:
+            return ops.painn_message_edges(graph.row_ptr, graph.dst32, r_ij, x_a, x_v, *actv_mlp, *dist_mlp, self.r0,
+                                           self.epsilon, residual)
         actv = self.mlp_actv(flat_a)
+        if dist_mlp is None or not fold:
+            out_a, out_v = ops.painn_message(graph.row_ptr, graph.dst32, r_ij, self.filters(r_ij), actv, flat_v, self.epsilon,
+                                             res_a, res_v)
+            return out_a.reshape(B, N, n), out_v.reshape(B, N, n, 3)
         # the filter's last layer runs inside the edge kernel: the (edges, 4n) filter is never stored
         first, second = self.mlp_dist.layers[0], self.mlp_dist.layers[2]
         if ops.painn_filter_hidden_supported(self.n_rbf, second.out_features, E):

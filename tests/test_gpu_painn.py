@@ -582,3 +582,75 @@ def test_update_elementwise_kernels_in_both_layouts(ops, rows, n):
         assert torch.equal(a, b)
     with pytest.raises(RuntimeError, match="lrv must have shape"):
         ops.painn_update_pre(torch.zeros(rows, 3 * n + 1, 3, device="cuda"), x_a.cuda())
+
+
+class _Scaled(torch.nn.Module):
+    """Another module in a submodule's place: a multiple of what that gives."""
+
+    def __init__(self, inner, factor):
+        super().__init__()
+        self.inner, self.factor = inner, factor
+
+    def forward(self, *args, **kwargs):
+        return self.factor * self.inner(*args, **kwargs)
+
+
+@pytest.mark.parametrize("how", ["hook", "replaced", "no bias"])
+@pytest.mark.parametrize("form", ["every edge", "grid", "folded", "training"])
+def test_submodules_are_called_where_a_call_is_more_than_their_parameters(pkg, how, form):
+    """Forward hooks on the MLPs, the norm and the maps of a PaiNN layer run and their results are used, another module in a
+    submodule's place is called, and a linear may have no bias: the layer gives what one with those changes written into its
+    weights gives, in each of the ways the message is evaluated and under autograd."""
+    import copy
+    painn = importlib.import_module("learned-dynamics_amd.painn")
+    gl = importlib.import_module("learned-dynamics_amd.graph_layers")
+    torch.manual_seed(0x947)
+    n, N = 64, 60
+    E = {"every edge": 300, "grid": 9000, "folded": 40000, "training": 500}[form]
+    training = form == "training"
+    src, dst = torch.sort(torch.randint(0, N, (E,))).values, torch.randint(0, N, (E,))
+    graph = gl.Graph(src.cuda(), dst.cuda(), None, 1, N)
+    x_a, x_v, r = torch.randn(1, N, n).cuda(), torch.randn(1, N, n, 3).cuda(), torch.randn(E, 3).cuda()
+    block = painn.Block(5.0, n, n_rbf=16).cuda().requires_grad_(training)
+    block.message.use_table = form == "grid"
+    want = copy.deepcopy(block)
+    calls = []
+    # under autograd the fused functions have always read the MLPs' and the norm's parameters: the maps are what is called
+    names = ["update.lin_l", "update.lin_r", "update.lin_v"] if training else ["message.mlp_actv", "message.mlp_dist", "update.mlp", "update.gn"]
+    for name in names:
+        module, twin = block.get_submodule(name), want.get_submodule(name)
+        parent, _, leaf = name.rpartition(".")
+        if how == "no bias":
+            if not isinstance(module, painn.MLP):
+                continue
+            module.layers[4] = torch.nn.Linear(n if "actv" in name else 4 * n, 1, bias=False).cuda().requires_grad_(False)
+            module.layers[4].weight = torch.nn.Parameter(twin.layers[4].weight.clone(), requires_grad=training)
+            with torch.no_grad():
+                twin.layers[4].bias.zero_()
+            continue
+        factor = 1.0 if name == "update.gn" else 2.0                         # (the norm's call adds operands that stay)
+        with torch.no_grad():
+            for p in (twin.layers[4].parameters() if isinstance(twin, painn.MLP) else twin.parameters()):
+                p.mul_(factor)
+        if how == "hook":
+            module.register_forward_hook(lambda m, args, out, name=name, k=factor: (calls.append(name), k * out)[1])
+        elif not (name == "message.mlp_dist" and form == "grid"):          # (another module there gets the MLP on every edge)
+            setattr(block.get_submodule(parent), leaf, _Scaled(module, factor))
+        else:
+            module.layers[4] = copy.deepcopy(twin.layers[4])
+    if how == "no bias" and training:
+        block.update.mlp.layers[4].bias = None
+        with torch.no_grad():
+            want.update.mlp.layers[4].bias.zero_()
+    inputs = (None, graph, r, None, None, x_a.requires_grad_(training), x_v.requires_grad_(training), None)
+    got_a, got_v = block(inputs)[5:7]
+    want_a, want_v = want(inputs)[5:7]
+    if how == "hook":
+        assert set(calls) == set(names)
+    # (both are fp32 layers of sums of at most 4 n terms: their distance is that of two orders of summation)
+    for a, b, what in ((got_a, want_a, "x_a"), (got_v, want_v, "x_v")):
+        torch.testing.assert_close(a, b, rtol=0, atol=2e-5 * float(b.abs().max()), msg=lambda m, what=what: f"{what}: {m}")
+    if training:
+        grads = [torch.autograd.grad((a ** 2).sum() + (v ** 2).sum(), (x_a, x_v)) for a, v in ((got_a, got_v), (want_a, want_v))]
+        for a, b in zip(*grads):
+            torch.testing.assert_close(a, b, rtol=0, atol=2e-5 * float(b.abs().max()))
