@@ -54,7 +54,7 @@ def plain_call(module, cls):
     hooks, no compiled call.  What the fused functions, which read a submodule's parameters and enqueue, may stand for."""
     own = module.__dict__
     return (type(module) is cls and "forward" not in own and own.get("_compiled_call_impl") is None
-            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+            and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
                      or _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks
                      or _nn_module._global_backward_hooks or _nn_module._global_backward_pre_hooks))
 
