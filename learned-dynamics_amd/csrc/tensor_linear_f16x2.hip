@@ -257,7 +257,7 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
     const long ld_row = my_row < R ? my_row : R - 1;
     const float* xrow = X + ld_row * I + 16 * g;
     float sx;
-    bool odd_cols, odd;                                      // this wave has columns, or anything, that the pieces cannot carry
+    bool odd;                                                // this wave has rows (columns: below) that the pieces cannot carry
     {
         float amax = 0.f;
         const float* xm = xmax + (ld_row / xmax_div) * xmax_stride;
@@ -266,13 +266,7 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
         float inv;
         sx = pow2_scale(amax, &inv);
         if (g == 0) inv_sx[wave * 32 + m] = beyond_split(amax) ? __builtin_nanf("") : inv;
-        const int* marked = marked_blocks(w_inv, O_pad) + n0 / 32;
-        int any = 0;
-#pragma unroll
-        for (int ni = 0; ni < NI; ni++) any |= marked[ni];   // (scalar loads)
-        asm volatile("" : "+s"(any));                        // (here, where others are waited for anyway, not in the epilogue)
-        odd_cols = any != 0;
-        odd = odd_cols || __any(beyond_split(amax));
+        odd = __any(beyond_split(amax));
     }
     const _Float16* wsrc[kPer];
     int wdst[kPer];
@@ -334,9 +328,15 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
     WRegs w;
     load_w(w, 0);
     load_a(a0, 0);
+    int marked = 0;
+#pragma unroll
+    for (int ni = 0; ni < NI; ni++) marked |= marked_blocks(w_inv, O_pad)[n0 / 32 + ni];      // (scalar loads)
     store_w(w, buf0);
     load_w(w, kCK);
     load_a(a1, kCK);
+    asm volatile("" : "+s"(marked));                         // (arrived by here, where W was waited for, and not in the epilogue)
+    const bool odd_cols = marked != 0;
+    odd |= odd_cols;
     __syncthreads();
     // chunks in pairs (even chunk: a0 / buf0, odd chunk: a1 / buf1); with an odd chunk count the
     // surplus chunk (a clamped reload of the last one) is scaled by zero instead of being branched
@@ -644,9 +644,12 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
         const int n = n0 + col;
         float v = 0.f;
         if (r < R && n < O) {
-            const long row = r / out_T;
-            const long addr = (row * O + n) * out_T + (r - row * out_T);
             const float isx = inv_sx[rl], iw = w_inv[n], bv = bias && r < bias_rows ? bias[n] : 0.f;
+            long addr = r * O + n;
+            if (out_T != 1) {                                 // (uniform)
+                const long row = r / out_T;
+                addr = (row * O + n) * out_T + (r - row * out_T);
+            }
             if (isx == isx && iw == iw) {
                 v = activate(sum * isx * iw + bv, act);
                 if (accumulate) v += Y[addr];
