@@ -9,6 +9,7 @@
 // split-fp16 linears scale by come out of the pass that writes the rows.
 // DUAL = false: no tangents (R rows); the tangent operands are ignored.
 #include "common.hpp"
+#include <algorithm>
 
 namespace mg {
 namespace {
@@ -481,7 +482,7 @@ constexpr int kPiece = 4096, kPieceStats = 5;      // count, mean, m2, mean of t
 template <bool DUAL>
 __global__ void __launch_bounds__(256) gn_pieces_kernel(const float* __restrict__ ip, const float* __restrict__ y, long R, int N,
                                                         int n, int groups, int pieces, float* __restrict__ part) {
-    const int piece = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
+    const int bg = blockIdx.x / pieces, piece = blockIdx.x - bg * pieces, b = bg / groups, g = bg - b * groups;
     const int cpg = n / groups;
     const long total = (long)N * cpg, lo = (long)piece * kPiece, hi = min(lo + kPiece, total);
     __shared__ float red[2][4];
@@ -619,7 +620,7 @@ __global__ void __launch_bounds__(256) gn_grad_pieces_kernel(const float* __rest
                                                              const GroupStats* __restrict__ stats, const float* __restrict__ g_a,
                                                              const float* __restrict__ g_at, long R, int N, int n, int groups,
                                                              int pieces, float* __restrict__ part) {
-    const int piece = blockIdx.x, b = blockIdx.y;
+    const int b = blockIdx.x / pieces, piece = blockIdx.x - b * pieces;
     const int cpg = n / groups;
     const int lo = piece * kGradNodes, hi = min(lo + kGradNodes, N);
     __shared__ float red[256 * kGradSums];
@@ -794,7 +795,7 @@ __global__ void __launch_bounds__(256) update_post_bwd_kernel(const float* __res
 // sums of gamma-weighted channel sums per group: (box, group, 5)
 __global__ void __launch_bounds__(64) gn_grad_groups_kernel(const float* __restrict__ sums, const float* __restrict__ gamma,
                                                             int n, int groups, float* __restrict__ out) {
-    const int g = blockIdx.x, b = blockIdx.y, cpg = n / groups;
+    const int b = blockIdx.x / groups, g = blockIdx.x - b * groups, cpg = n / groups;
 #pragma unroll
     for (int q = 0; q < kGradSums; q++) {
         float acc = 0.f;
@@ -914,7 +915,7 @@ int mg_silu_rows_bwd(const float* z, const float* dh, long rows, int n, int dual
 int mg_painn_edge_encode_fwd(const float* r, const float* r_t, long E, int n, float rmax, float eps, float* enc, float* enc_bound,
                              float* dir, float* dir_t, mg_stream_t stream) {
     const bool dual = r_t != nullptr;
-    MG_REQUIRE(E >= 0 && n >= 1 && rmax > 0.f && eps > 0.f, "mg_painn_edge_encode_fwd: bad argument");
+    MG_REQUIRE(E >= 0 && n >= 1 && rmax > 0.f, "mg_painn_edge_encode_fwd: bad argument");
     if (E == 0) return MG_OK;
     MG_REQUIRE(r && enc && enc_bound && dir && (!dual || dir_t), "mg_painn_edge_encode_fwd: null pointer");
     const int lanes = row_lanes(n);
@@ -926,7 +927,7 @@ int mg_painn_edge_encode_fwd(const float* r, const float* r_t, long E, int n, fl
 int mg_painn_edge_encode_bwd(const float* r, const float* r_t, long E, int n, float rmax, float eps, const float* g_enc,
                              const float* g_dir, const float* g_dir_t, float* g_r, float* g_r_t, mg_stream_t stream) {
     const bool dual = r_t != nullptr;
-    MG_REQUIRE(E >= 0 && n >= 1 && rmax > 0.f && eps > 0.f, "mg_painn_edge_encode_bwd: bad argument");
+    MG_REQUIRE(E >= 0 && n >= 1 && rmax > 0.f, "mg_painn_edge_encode_bwd: bad argument");
     if (E == 0) return MG_OK;
     MG_REQUIRE(r && g_enc && g_dir && g_r && (!dual || (g_dir_t && g_r_t)), "mg_painn_edge_encode_bwd: null pointer");
     const int lanes = row_lanes(n);
@@ -1002,15 +1003,16 @@ int mg_painn_update_post_fwd(const float* lrv, const float* ip, const float* y, 
                              int nodes, int n, int groups, float eps, int dual, float* scratch, float* stats, float* out_a,
                              float* out_v, mg_stream_t stream) {
     const long R = (long)batch * nodes;
-    MG_REQUIRE(batch >= 0 && nodes >= 0 && batch <= 65535 && groups >= 1 && groups <= 65535 && rows_ok(R, n) && n % groups == 0,
+    MG_REQUIRE(batch >= 0 && nodes >= 0 && groups >= 1 && rows_ok(R, n) && n % groups == 0,
                "mg_painn_update_post_fwd: bad shape");
     if (R == 0) return MG_OK;
     MG_REQUIRE(lrv && ip && y && gamma && beta && scratch && stats && out_a && out_v && aligned16(lrv) && aligned16(ip) &&
                    aligned16(y) && aligned16(out_a) && aligned16(out_v) && aligned16(stats),
                "mg_painn_update_post_fwd: null or unaligned pointer");
     const int pieces = (int)ceil_div((long)nodes * (n / groups), kPiece);
+    MG_REQUIRE((long)pieces * groups * batch <= 0x7fffffffL, "mg_painn_update_post_fwd: too many boxes");
     GroupStats* st = reinterpret_cast<GroupStats*>(stats);
-    MG_DUAL_LAUNCH(gn_pieces_kernel, dim3(pieces, groups, batch), dim3(256), ip, y, R, nodes, n, groups, pieces, scratch);
+    MG_DUAL_LAUNCH(gn_pieces_kernel, dim3((unsigned)(pieces * groups * batch)), dim3(256), ip, y, R, nodes, n, groups, pieces, scratch);
     hipLaunchKernelGGL(gn_finish_kernel, dim3((unsigned)(batch * groups)), dim3(64), 0, (hipStream_t)stream, scratch, pieces, eps, st);
     MG_DUAL_LAUNCH(update_post_fwd_kernel, dim3((unsigned)ceil_div(R * (n / 4), 256)), dim3(256), lrv, ip, y, st, gamma, beta, R,
                    nodes, n, groups, out_a, out_v);
@@ -1022,7 +1024,7 @@ int mg_painn_update_post_bwd(const float* lrv, const float* ip, const float* y, 
                              int groups, int dual, float* scratch, float* g_y, float* g_y_rowmax, float* g_ip, float* g_lrv,
                              float* d_gamma, float* d_beta, mg_stream_t stream) {
     const long R = (long)batch * nodes;
-    MG_REQUIRE(batch >= 1 && nodes >= 1 && batch <= 65535 && groups >= 1 && rows_ok(R, n) && n % groups == 0,
+    MG_REQUIRE(batch >= 1 && nodes >= 1 && groups >= 1 && rows_ok(R, n) && n % groups == 0,
                "mg_painn_update_post_bwd: bad shape");
     MG_REQUIRE(lrv && ip && y && stats && gamma && g_a && g_v && (!dual || (g_a_t && g_v_t)) && scratch && g_y && g_y_rowmax && g_ip &&
                    g_lrv && d_gamma && d_beta,
@@ -1031,14 +1033,15 @@ int mg_painn_update_post_bwd(const float* lrv, const float* ip, const float* y, 
                    aligned16(g_v) && aligned16(g_v_t) && aligned16(g_y) && aligned16(g_ip) && aligned16(g_lrv),
                "mg_painn_update_post_bwd: unaligned pointer");
     const int pieces = (int)ceil_div(nodes, kGradNodes);
+    MG_REQUIRE((long)std::max(pieces, groups) * batch <= 0x7fffffffL, "mg_painn_update_post_bwd: too many boxes");
     const GroupStats* st = reinterpret_cast<const GroupStats*>(stats);
     float* channel = scratch + (long)batch * pieces * kGradSums * n;
     float* group = channel + (long)batch * kGradSums * n;
     hipStream_t s = (hipStream_t)stream;
-    MG_DUAL_LAUNCH(gn_grad_pieces_kernel, dim3(pieces, batch), dim3(256), ip, y, st, g_a, g_a_t, R, nodes, n, groups, pieces, scratch);
+    MG_DUAL_LAUNCH(gn_grad_pieces_kernel, dim3((unsigned)(pieces * batch)), dim3(256), ip, y, st, g_a, g_a_t, R, nodes, n, groups, pieces, scratch);
     hipLaunchKernelGGL(gn_grad_finish_kernel, dim3((unsigned)n), dim3(64), 0, s, scratch, st, batch, n, groups, pieces, channel,
                        d_gamma, d_beta);
-    hipLaunchKernelGGL(gn_grad_groups_kernel, dim3(groups, batch), dim3(64), 0, s, channel, gamma, n, groups, group);
+    hipLaunchKernelGGL(gn_grad_groups_kernel, dim3((unsigned)(groups * batch)), dim3(64), 0, s, channel, gamma, n, groups, group);
     const int lanes = row_lanes(n);
     MG_DUAL_LAUNCH(update_post_bwd_kernel, dim3(row_blocks(R, lanes)), dim3(256), lrv, ip, y, st, group, gamma, g_a, g_a_t, g_v, g_v_t,
                    R, nodes, n, groups, lanes, g_y, g_y_rowmax, g_ip, g_lrv);
