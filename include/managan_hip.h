@@ -302,7 +302,8 @@ int mg_tensor_linear_packed(const void* packed_W, const float* x, long rows, int
                             mg_stream_t stream);
 /* Mode 2: two-piece fp16 split with per-row power-of-two scales, three fp16 MFMAs per product,
  * fp32 accumulation (a few fp32 ulps per product; half the matrix work of mode 1).
- * mg_linear_f16x2_pack_weight: W -> hi / lo fp16 planes (dim_out rounded up to 256 rows) followed by
+ * mg_linear_f16x2_pack_weight: W (dim_in % 8 == 0; zero columns up to a multiple of 32) -> hi / lo fp16
+ * planes (dim_out rounded up to 256 rows) followed by
  * one fp32 inverse scale per row (a NaN where the row holds an infinity or NaN) and one flag per 32 rows,
  * in caller-owned memory of mg_linear_f16x2_packed_weight_bytes bytes.
  * mg_tensor_linear_f16x2: y = act(x W^T + bias) for plain rows x (rows, dim_in), dim_in % 32 == 0;

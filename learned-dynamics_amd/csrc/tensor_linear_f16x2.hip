@@ -682,6 +682,7 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
 }
 
 inline int o_pad_of(int dim_out) { return (dim_out + 255) / 256 * 256; }
+inline int i_pad_of(int dim_in) { return (dim_in + 31) / 32 * 32; }
 
 // The split-K kernel is for problems whose row-streaming tiles would leave most of the chip idle while a few workgroups walk
 // K one barrier at a time.  The rule is the measured crossover (R = 337 .. 49152, K = 128 .. 1280, O = 64 .. 512) in units
@@ -761,7 +762,7 @@ extern "C" {
 int mg_linear_f16x2_packed_weight_bytes(int dim_in, int dim_out, size_t* bytes) {
     MG_REQUIRE(bytes != nullptr && dim_in >= 0 && dim_out >= 0, "mg_linear_f16x2_packed_weight_bytes: bad argument");
     const size_t o_pad = (size_t)o_pad_of(dim_out);
-    *bytes = 2 * o_pad * (size_t)dim_in * sizeof(_Float16) + o_pad * sizeof(float) + o_pad / 32 * sizeof(int);
+    *bytes = 2 * o_pad * (size_t)i_pad_of(dim_in) * sizeof(_Float16) + o_pad * sizeof(float) + o_pad / 32 * sizeof(int);
     return MG_OK;
 }
 
@@ -782,7 +783,7 @@ int mg_linear_f16x2_pack_weights(const mg_f16x2_weight* weights, int count, mg_s
         MG_REQUIRE(w.dim_in >= 0 && w.dim_out >= 0 && w.dim_pad >= w.dim_in, "mg_linear_f16x2_pack_weight: bad size");
         if (w.dim_in == 0 || w.dim_out == 0) continue;
         MG_REQUIRE(w.W && w.packed && aligned16(w.packed), "mg_linear_f16x2_pack_weight: null or unaligned pointer");
-        MG_REQUIRE(w.dim_pad % 32 == 0, "mg_linear_f16x2_pack_weight: dim_in must be a multiple of 32");
+        MG_REQUIRE(w.dim_pad % 32 == 0, "mg_linear_f16x2_pack_weight: dim_pad must be a multiple of 32");
         const int O_pad = o_pad_of(w.dim_out);
         jobs.job[jobs.count++] = PackJob{w.W, w.stride_o, w.stride_i, w.dim_in, w.dim_pad, w.dim_out, O_pad, blocks,
                                          static_cast<_Float16*>(w.packed)};
@@ -801,7 +802,8 @@ int mg_linear_f16x2_pack_weight_padded(const float* W, long w_stride_o, long w_s
 
 int mg_linear_f16x2_pack_weight(const float* W, long w_stride_o, long w_stride_i, int dim_in, int dim_out,
                                 void* packed, mg_stream_t stream) {
-    return mg_linear_f16x2_pack_weight_padded(W, w_stride_o, w_stride_i, dim_in, dim_out, dim_in, packed, stream);
+    MG_REQUIRE(dim_in % 8 == 0, "mg_linear_f16x2_pack_weight: dim_in must be a multiple of 8");
+    return mg_linear_f16x2_pack_weight_padded(W, w_stride_o, w_stride_i, dim_in, dim_out, i_pad_of(dim_in), packed, stream);
 }
 
 int mg_row_absmax(const float* x, long rows, int dim, float* out, mg_stream_t stream) {

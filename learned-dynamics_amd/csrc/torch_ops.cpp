@@ -111,7 +111,9 @@ at::Tensor packed_bf16x3(const at::Tensor& W) {
 at::Tensor packed_weight(const at::Tensor& W, bool f16) {
     TORCH_CHECK(W.is_cuda() && W.scalar_type() == at::kFloat && W.dim() == 2, "W must be a float32 CUDA matrix");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(W.device());
-    return f16 ? packed_f16x2(W, W.size(1)) : packed_bf16x3(W);
+    if (!f16) return packed_bf16x3(W);
+    TORCH_CHECK(W.size(1) % 8 == 0, "packed_weight_f16x2: dim_in must be a multiple of 8");
+    return packed_f16x2(W, (W.size(1) + 31) / 32 * 32);
 }
 
 // (max_o sum_i |W[o, i]|, max_o |bias[o]|): |act(x W^T + bias)| <= |x|max * first + second for |act(z)| <= |z|; read back

@@ -740,3 +740,13 @@ def test_small_problems_are_no_less_precise_than_fp32(ops, inds, rows, dim_in, d
     finally:
         ops.set_linear_mode(ops.LINEAR_F16X2)
     assert default <= 1.01 * fp32, (default, fp32)               # (where both run the same kernel they are equal)
+
+
+def test_packed_weight_of_any_multiple_of_eight(ops):
+    """A reduction of 8, 40 or 72 packs as with zero columns up to the next multiple of 32; 12 is refused."""
+    for dim_in in (8, 40, 72):
+        W = torch.randn(50, dim_in, device="cuda")
+        padded = torch.nn.functional.pad(W, (0, -dim_in % 32))
+        assert torch.equal(ops.packed_weight_f16x2(W), ops.packed_weight_f16x2(padded))
+    with pytest.raises(RuntimeError, match="multiple of 8"):
+        ops.packed_weight_f16x2(torch.randn(50, 12, device="cuda"))
