@@ -5,11 +5,13 @@
 #include "torch_common.hpp"
 
 #include <atomic>
+#include <climits>
 #include <map>
 #include <mutex>
 #include <tuple>
 
 using namespace mgt;
+namespace py = pybind11;
 
 namespace {
 
@@ -21,7 +23,8 @@ std::atomic<int64_t> g_epoch{0};        // of invalidate_weight_caches
 // ------------------------------------------------------------------ tensors derived from weights, kept per version
 // An entry belongs to a tensor OBJECT (a weak reference keeps the address from being reused) and its version counter;
 // a view (the transposed weight of an input-gradient product is a fresh view of the parameter) is kept under the tensor
-// it views.  Inference tensors have no version counter: nothing is kept for them.
+// it views.  It goes when that tensor does: a Python weak reference to it says when.  Inference tensors have no version
+// counter: nothing is kept for them.  (Callers hold the GIL.)
 template <typename Value>
 class WeightCache {
 public:
@@ -61,18 +64,43 @@ public:
                 return it->second.value;
         }
         Value v = make();
+        watch(owner, impl);
+        Slot slot{c10::weak_intrusive_ptr<c10::TensorImpl>(owner.getIntrusivePtr()), version, data, epoch, v};
         std::lock_guard<std::mutex> lock(mutex_);
-        if (++inserts_ % 64 == 0 || slots_.size() > 8192)          // drop what belonged to tensors that are gone
-            for (auto it = slots_.begin(); it != slots_.end();) it = it->second.owner.expired() ? slots_.erase(it) : std::next(it);
-        slots_.erase(key);
-        slots_.emplace(key, Slot{c10::weak_intrusive_ptr<c10::TensorImpl>(owner.getIntrusivePtr()), version, data, epoch, v});
+        auto it = slots_.find(key);
+        if (it == slots_.end()) slots_.emplace(key, std::move(slot));
+        else std::swap(it->second, slot);                     // (the old value goes with `slot`, after the lock)
         return v;
     }
 
 private:
+    void watch(const at::Tensor& owner, c10::TensorImpl* impl) {
+        {
+            std::lock_guard<std::mutex> lock(mutex_);
+            if (watched_.count(impl)) return;
+        }
+        py::object obj = py::cast(owner);
+        py::weakref ref(obj, py::cpp_function([this, impl](py::object) { forget(impl); }));
+        std::lock_guard<std::mutex> lock(mutex_);
+        watched_.emplace(impl, std::move(ref));
+    }
+    void forget(c10::TensorImpl* impl) {
+        std::vector<Slot> gone;                               // (destroyed after the lock: what they free may call back)
+        py::object ref;
+        std::lock_guard<std::mutex> lock(mutex_);
+        for (auto it = slots_.lower_bound(Key{impl, INT_MIN, INT64_MIN, INT64_MIN, INT64_MIN, INT64_MIN, INT64_MIN, INT64_MIN});
+             it != slots_.end() && std::get<0>(it->first) == impl; it = slots_.erase(it))
+            gone.push_back(std::move(it->second));
+        auto w = watched_.find(impl);
+        if (w != watched_.end()) {
+            ref = std::move(w->second);
+            watched_.erase(w);
+        }
+    }
+
     std::mutex mutex_;
     std::map<Key, Slot> slots_;
-    int64_t inserts_ = 0;
+    std::map<const void*, py::object> watched_;
 };
 
 template <typename Value>
@@ -161,10 +189,11 @@ int64_t rowmax_parts(int64_t rows, int64_t dim_in, int64_t dim_out, bool sequent
                       : mg_tensor_linear_f16x2_rowmax_parts(rows, (int)dim_in, (int)dim_out);
 }
 
-// x (rows, k) plain rows; y preallocated
+// x (rows, k) plain rows; y preallocated; packed: W's planes where the caller holds them
 void run_f16x2(const at::Tensor& W, int64_t k, const float* x, int64_t rows, const Bound& b, const OptTensor& bias, int act,
-               bool accumulate, int out_comps, at::Tensor& y, at::Tensor* ymax, bool sequential, int64_t bias_rows = -1) {
-    const at::Tensor planes = packed_f16x2(W, k);
+               bool accumulate, int out_comps, at::Tensor& y, at::Tensor* ymax, bool sequential, int64_t bias_rows = -1,
+               const OptTensor& packed = OptTensor()) {
+    const at::Tensor planes = packed.has_value() ? *packed : packed_f16x2(W, k);
     const at::Tensor& base = *b.base;
     mg_f16x2_linear a{};
     a.packed_W = planes.data_ptr();
@@ -659,15 +688,21 @@ at::Tensor stacked(const at::Tensor& p, const OptTensor& t, int64_t cols) {
     return at::cat({p.reshape({rows, cols}), t->reshape({rows, cols})});
 }
 
-// packed planes of several weights that the next kernels read, those that are missing in one launch
-void pack_ahead(const Tensors& weights) {
-    if (mg_get_linear_mode() != kModeF16x2) return;
-    Tensors missing;
+bool packs_f16x2(const at::Tensor& W) { return W.size(1) % 32 == 0 && W.size(1) >= 64 && W.size(0) >= 8; }
+
+// Packed planes of several weights that the next kernels read, those that are missing in one launch.  `passing`: weights that
+// do not outlive this pass; their planes are returned and not kept.
+std::vector<OptTensor> pack_ahead(const Tensors& weights, const Tensors& passing = {}) {
+    std::vector<OptTensor> out(passing.size());
+    if (mg_get_linear_mode() != kModeF16x2) return out;
+    Tensors missing, planes;
     for (const at::Tensor& W : weights)
-        if (W.size(1) % 32 == 0 && W.size(1) >= 64 && W.size(0) >= 8 && !cache<at::Tensor>().has(W, 2, W.size(1))) missing.push_back(W);
-    if (missing.size() < 2) return;
+        if (packs_f16x2(W) && !cache<at::Tensor>().has(W, 2, W.size(1))) missing.push_back(W);
+    const size_t kept = missing.size();
+    for (const at::Tensor& W : passing)
+        if (packs_f16x2(W)) missing.push_back(W);
+    if (missing.size() < 2 && kept == missing.size()) return out;
     std::vector<mg_f16x2_weight> jobs;
-    Tensors planes;
     for (const at::Tensor& W : missing) {
         size_t bytes = 0;
         check(mg_linear_f16x2_packed_weight_bytes((int)W.size(1), (int)W.size(0), &bytes));
@@ -676,20 +711,24 @@ void pack_ahead(const Tensors& weights) {
                         planes.back().data_ptr()});
     }
     check(mg_linear_f16x2_pack_weights(jobs.data(), (int)jobs.size(), stream_of(missing[0])));
-    for (size_t k = 0; k < missing.size(); k++) {
+    for (size_t k = 0; k < kept; k++) {
         const at::Tensor p = planes[k];
         cache<at::Tensor>().get(missing[k], 2, missing[k].size(1), [&] { return p; });
     }
+    for (size_t k = 0, at = kept; k < passing.size(); k++)
+        if (packs_f16x2(passing[k])) out[k] = planes[at++];
+    return out;
 }
 
 // y = x W^T, with the bias added to the first bias_rows rows
-at::Tensor rows_linear(const at::Tensor& W, const OptTensor& bias, const at::Tensor& x, int64_t bias_rows, Bound bound) {
+at::Tensor rows_linear(const at::Tensor& W, const OptTensor& bias, const at::Tensor& x, int64_t bias_rows, Bound bound,
+                       const OptTensor& packed = OptTensor()) {
     const int64_t rows = x.size(0), dim_in = W.size(1), dim_out = W.size(0);
     at::Tensor y = floats(x, {rows, dim_out});
     if (rows == 0) return y;
     if (mg_get_linear_mode() == kModeF16x2 && f16x2_takes(rows, dim_in, dim_out, x)) {
         if (!bound.base.has_value()) bound = Bound{row_absmax(x)};
-        run_f16x2(W, dim_in, fp(x), rows, bound, bias, kActNone, false, 1, y, nullptr, false, bias_rows);
+        run_f16x2(W, dim_in, fp(x), rows, bound, bias, kActNone, false, 1, y, nullptr, false, bias_rows, packed);
         return y;
     }
     auto piece = [&](int64_t lo, int64_t hi, const OptTensor& b) {
@@ -924,9 +963,9 @@ std::tuple<Tensors, std::vector<OptTensor>> painn_update_train_fwd(const at::Ten
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x_a.device());
     const int64_t copies = dual ? 2 : 1;
     const at::Tensor W_lrv = at::cat(lrv_W);
-    pack_ahead({W_lrv, W_lrv.t(), W[0], W[1], W[2], W[0].t(), W[1].t(), W[2].t()});
+    const auto lrv_planes = pack_ahead({W[0], W[1], W[2], W[0].t(), W[1].t(), W[2].t()}, {W_lrv, W_lrv.t()});
     auto [x2, x2max] = vector_rows(x_v, x_vt, R, n);
-    const at::Tensor lrv = rows_linear(W_lrv, OptTensor(), x2, 0, Bound{OptTensor(x2max)});
+    const at::Tensor lrv = rows_linear(W_lrv, OptTensor(), x2, 0, Bound{OptTensor(x2max)}, lrv_planes[0]);
     at::Tensor ip = floats(x_a, {copies * R, n}), cat = floats(x_a, {copies * R, 2 * n}), cat_max = floats(x_a, {copies * R, 1});
     const mg_stream_t st = stream_of(x_a);
     check(mg_painn_update_pre_fwd(fp(lrv), fp(x_a), fp(x_at), R, (int)n, dual, fp(ip), fp(cat), fp(cat_max), st));
@@ -944,7 +983,7 @@ std::tuple<Tensors, std::vector<OptTensor>> painn_update_train_fwd(const at::Ten
         out.push_back(*second_half(out_v, x_v.sizes(), true));
     }
     std::vector<OptTensor> saved{OptTensor(W_lrv), OptTensor(x2), OptTensor(x2max), OptTensor(lrv), OptTensor(ip), OptTensor(cat),
-                                 OptTensor(y), OptTensor(stats)};
+                                 OptTensor(y), OptTensor(stats), lrv_planes[1]};
     saved.insert(saved.end(), mlp_saved.begin(), mlp_saved.end());
     return {out, saved};
 }
@@ -962,7 +1001,7 @@ std::tuple<std::vector<OptTensor>, Tensors> painn_update_train_bwd(const at::Ten
     c10::hip::HIPGuardMasqueradingAsCUDA guard(g_a.device());
     const at::Tensor &W_lrv = *saved[0], &x2 = *saved[1], &lrv = *saved[3], &ip = *saved[4], &cat = *saved[5], &y = *saved[6],
                      &stats = *saved[7];
-    const std::vector<OptTensor> mlp_saved(saved.begin() + 8, saved.end());
+    const std::vector<OptTensor> mlp_saved(saved.begin() + 9, saved.end());
     const mg_stream_t st = stream_of(g_a);
     long fwd = 0, bwd = 0;
     check(mg_painn_update_scratch_floats((int)B, (int)N, (int)n, groups, &fwd, &bwd));
@@ -982,7 +1021,8 @@ std::tuple<std::vector<OptTensor>, Tensors> painn_update_train_bwd(const at::Ten
     const at::Tensor back = W_lrv.t();
     if (mg_get_linear_mode() == kModeF16x2 && f16x2_takes(copies * R * 3, 3 * n, n, g_lrv)) {
         g_xv = floats(g_a, {copies * R, n, 3});
-        run_f16x2(back, 3 * n, fp(g_lrv), copies * R * 3, Bound{g_bound}, OptTensor(), kActNone, false, 3, g_xv, nullptr, false);
+        run_f16x2(back, 3 * n, fp(g_lrv), copies * R * 3, Bound{g_bound}, OptTensor(), kActNone, false, 3, g_xv, nullptr, false, -1,
+                  saved[8]);
     } else {
         g_xv = rows_linear(back, OptTensor(), g_lrv, 0, Bound{g_bound}).reshape({copies * R, 3, n}).transpose(1, 2).contiguous();
     }
@@ -1119,7 +1159,6 @@ std::tuple<Tensors, OptTensor, OptTensor> bee_message_bwd(const Tensors& left, c
 }  // namespace
 
 void register_ops(pybind11::module_& m) {
-    namespace py = pybind11;
     m.def("invalidate_weight_caches", [] { g_epoch.fetch_add(1); });
     m.def("packed_weight", &packed_weight);
     m.def("row_absmax", &row_absmax);

@@ -167,3 +167,42 @@ def test_tensor_prods_equals_the_ctypes_route_and_the_module_uses_it(ext, ops, i
         ext.tensor_prods(*inds, W_l, W_r, W_o, x_l[:2], x_r)
     with pytest.raises(RuntimeError, match="float32 CUDA"):
         ext.tensor_prods(*inds, W_l, W_r, W_o, x_l.cpu(), x_r)
+
+
+def test_planes_go_with_the_weight_they_were_packed_from(ops):
+    """Packed planes are freed when their weight is deleted (not at some later packing), those of a transposed view with the
+    weight it views, and a weight that stays keeps its own."""
+    keep = torch.randn(256, 256, device="cuda")
+    planes = ops.packed_weight_f16x2(keep)
+    x = torch.randn(40, 256, device="cuda")
+    ops.tensor_linear_fwd(0, keep.t(), x)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    for _ in range(3):
+        W = torch.randn(512, 256, device="cuda")
+        ops.packed_weight_f16x2(W)
+        y = ops.tensor_linear_fwd(0, W.t(), torch.randn(40, 512, device="cuda"))
+        view = W.t()
+        del W, y
+        assert torch.cuda.memory_allocated() >= before + 3 * 512 * 256 * 4          # the view keeps the weight and its planes
+        del view
+        assert torch.cuda.memory_allocated() == before
+    assert ops.packed_weight_f16x2(keep).data_ptr() == planes.data_ptr()
+
+
+def test_a_training_step_leaves_no_planes_behind(pkg):
+    """The stacked maps of the update are weights of one pass: their planes go with it."""
+    painn = importlib.import_module("learned-dynamics_amd.painn")
+    torch.manual_seed(0x947)
+    upd = painn.Update(64).cuda()
+    opt = torch.optim.SGD(upd.parameters(), lr=1e-3)
+    x_a, x_v = torch.randn(1, 300, 64, device="cuda"), torch.randn(1, 300, 64, 3, device="cuda")
+    held = []
+    for _ in range(6):
+        a, v = upd(x_a, x_v)
+        opt.zero_grad(set_to_none=True)
+        ((a ** 2).sum() + (v ** 2).sum()).backward()
+        opt.step()
+        del a, v
+        held.append(torch.cuda.memory_allocated())
+    assert len(set(held[1:])) == 1, held
