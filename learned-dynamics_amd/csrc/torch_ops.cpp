@@ -145,22 +145,27 @@ at::Tensor packed_weight(const at::Tensor& W, bool f16) {
 }
 
 // (max_o sum_i |W[o, i]|, max_o |bias[o]|): |act(x W^T + bias)| <= |x|max * first + second for |act(z)| <= |z|; read back
-// once per version of the parameters
+// once per version of the parameters, both with one copy, other Python threads running meanwhile
 std::pair<float, float> norms_of(const at::Tensor& W, const OptTensor& bias) {
-    auto read = [](const at::Tensor& t) { return t.item<float>(); };
-    auto weight = cache<float>().get(W, 3, 0, [&] {
-        c10::InferenceMode off(false);
-        at::NoGradGuard no_grad;
-        return read(W.detach().abs().sum(1).amax()) * (1.0f + 1e-6f);
-    });
-    float b = 0.f;
-    if (bias.has_value())
-        b = cache<float>().get(*bias, 4, 0, [&] {
-            c10::InferenceMode off(false);
-            at::NoGradGuard no_grad;
-            return read(bias->detach().abs().amax()) * (1.0f + 1e-6f);
-        });
-    return {weight, b};
+    auto read = [](std::vector<at::Tensor> t) {
+        const at::Tensor stacked = at::stack(t);
+        py::gil_scoped_release release;
+        const at::Tensor host = stacked.cpu();
+        std::pair<float, float> v{host.data_ptr<float>()[0], host.numel() > 1 ? host.data_ptr<float>()[1] : 0.f};
+        return v;
+    };
+    c10::InferenceMode off(false);
+    at::NoGradGuard no_grad;
+    auto of_weight = [&] { return W.detach().abs().sum(1).amax(); };
+    auto of_bias = [&] { return bias->detach().abs().amax(); };
+    constexpr float kAbove = 1.0f + 1e-6f;                    // (the product with a row maximum must not round below the bound)
+    auto& kept = cache<float>();
+    if (bias.has_value() && !kept.has(W, 3, 0) && !kept.has(*bias, 4, 0)) {
+        const auto both = read({of_weight(), of_bias()});
+        return {kept.get(W, 3, 0, [&] { return both.first * kAbove; }), kept.get(*bias, 4, 0, [&] { return both.second * kAbove; })};
+    }
+    const float weight = kept.get(W, 3, 0, [&] { return read({of_weight()}).first * kAbove; });
+    return {weight, bias.has_value() ? kept.get(*bias, 4, 0, [&] { return read({of_bias()}).first * kAbove; }) : 0.f};
 }
 
 // ------------------------------------------------------------------ linear maps

@@ -206,3 +206,33 @@ def test_a_training_step_leaves_no_planes_behind(pkg):
         del a, v
         held.append(torch.cuda.memory_allocated())
     assert len(set(held[1:])) == 1, held
+
+
+def test_other_threads_run_while_the_norms_are_read_back(ops):
+    """The first call with new weights waits for the device; a Python thread beside it goes on meanwhile."""
+    import threading
+    W, b = [torch.randn(128, 128, device="cuda") for _ in range(2)], [torch.randn(128, device="cuda") for _ in range(2)]
+    x = torch.randn(64, 128, device="cuda")
+    ops.linear_chain(x, W, b, (ops.ACT_SILU, ops.ACT_NONE))                   # (everything loaded and allocated)
+    with torch.no_grad():
+        W[0].mul_(2.0)
+        b[0].mul_(2.0)
+    stamps, stop = [], threading.Event()
+
+    def tick():
+        while not stop.wait(1e-3):
+            stamps.append(time.perf_counter())
+
+    thread = threading.Thread(target=tick)
+    thread.start()
+    try:
+        torch.cuda._sleep(500_000_000)                                       # some 0.2 s of a busy device
+        began = time.perf_counter()
+        ops.linear_chain(x, W, b, (ops.ACT_SILU, ops.ACT_NONE))
+        ended = time.perf_counter()
+    finally:
+        stop.set()
+        thread.join()
+    if ended - began < 0.05:
+        pytest.skip("the device was not busy long enough")
+    assert sum(began < t < ended for t in stamps) > 10
