@@ -9,6 +9,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <unordered_map>
 
 using namespace mgt;
 namespace py = pybind11;
@@ -25,6 +26,8 @@ std::atomic<int64_t> g_epoch{0};        // of invalidate_weight_caches
 // a view (the transposed weight of an input-gradient product is a fresh view of the parameter) is kept under the tensor
 // it views.  It goes when that tensor does: a Python weak reference to it says when.  Inference tensors have no version
 // counter: nothing is kept for them.  (Callers hold the GIL.)
+void watch_owner(const at::Tensor& owner);       // entries of this tensor are forgotten when it goes
+
 template <typename Value>
 class WeightCache {
 public:
@@ -64,7 +67,7 @@ public:
                 return it->second.value;
         }
         Value v = make();
-        watch(owner, impl);
+        watch_owner(owner);
         Slot slot{c10::weak_intrusive_ptr<c10::TensorImpl>(owner.getIntrusivePtr()), version, data, epoch, v};
         std::lock_guard<std::mutex> lock(mutex_);
         auto it = slots_.find(key);
@@ -73,40 +76,55 @@ public:
         return v;
     }
 
-private:
-    void watch(const at::Tensor& owner, c10::TensorImpl* impl) {
-        {
-            std::lock_guard<std::mutex> lock(mutex_);
-            if (watched_.count(impl)) return;
-        }
-        py::object obj = py::cast(owner);
-        py::weakref ref(obj, py::cpp_function([this, impl](py::object) { forget(impl); }));
-        std::lock_guard<std::mutex> lock(mutex_);
-        watched_.emplace(impl, std::move(ref));
-    }
-    void forget(c10::TensorImpl* impl) {
+    void forget(const void* impl) {
         std::vector<Slot> gone;                               // (destroyed after the lock: what they free may call back)
-        py::object ref;
         std::lock_guard<std::mutex> lock(mutex_);
         for (auto it = slots_.lower_bound(Key{impl, INT_MIN, INT64_MIN, INT64_MIN, INT64_MIN, INT64_MIN, INT64_MIN, INT64_MIN});
              it != slots_.end() && std::get<0>(it->first) == impl; it = slots_.erase(it))
             gone.push_back(std::move(it->second));
-        auto w = watched_.find(impl);
-        if (w != watched_.end()) {
-            ref = std::move(w->second);
-            watched_.erase(w);
-        }
     }
 
+private:
     std::mutex mutex_;
     std::map<Key, Slot> slots_;
-    std::map<const void*, py::object> watched_;
 };
 
 template <typename Value>
 WeightCache<Value>& cache() {
     static WeightCache<Value>* c = new WeightCache<Value>;     // never destroyed: the allocator may be gone by then
     return *c;
+}
+
+// Python weak references to the tensors that have entries, with one callback for all of them (the GIL guards the maps)
+struct Owners {
+    py::object callback;
+    std::unordered_map<const void*, py::object> refs;         // tensor -> weak reference
+    std::unordered_map<PyObject*, const void*> tensors;       // weak reference -> tensor
+};
+Owners& owners() {
+    static Owners* o = new Owners;                             // never destroyed: tensors may outlive the interpreter's modules
+    return *o;
+}
+void owner_gone(py::object ref) {
+    Owners& o = owners();
+    auto it = o.tensors.find(ref.ptr());
+    if (it == o.tensors.end()) return;
+    const void* impl = it->second;
+    o.tensors.erase(it);
+    o.refs.erase(impl);
+    cache<at::Tensor>().forget(impl);
+    cache<float>().forget(impl);
+}
+void watch_owner(const at::Tensor& owner) {
+    Owners& o = owners();
+    const void* impl = owner.unsafeGetTensorImpl();
+    if (o.refs.count(impl)) return;
+    if (!o.callback) o.callback = py::cpp_function(&owner_gone);
+    py::object obj = py::cast(owner);
+    PyObject* ref = PyWeakref_NewRef(obj.ptr(), o.callback.ptr());
+    if (!ref) throw py::error_already_set();
+    o.tensors.emplace(ref, impl);
+    o.refs.emplace(impl, py::reinterpret_steal<py::object>(ref));
 }
 
 at::Tensor bytes_like(const at::Tensor& t, size_t n) {
