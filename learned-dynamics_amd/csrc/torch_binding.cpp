@@ -125,9 +125,10 @@ std::tuple<at::Tensor, at::Tensor> get_neighbours(int listmax, int neighboursmax
 }
 
 // The radius graph of Graph.radius_graph / graph_setup in one call.  The fill pass is queued before the edge count is
-// known, into arrays sized from an estimate (the count of the last search of this shape, else the mean density, plus a
-// margin), while the host polls the four statistics, which the kernel stores into pinned memory; only an estimate that
-// was too small costs a second pass.
+// known, into arrays sized from an estimate, while the host polls the four statistics, which the kernel stores into pinned
+// memory; only an estimate that was too small costs a second pass.  The arrays (36 bytes an edge) live as long as the graph,
+// so the margin is small: 12.5 % over the count of a uniform system in the first search of a shape, then 2.5 % over the largest
+// recent one (EdgeHints), which trajectories and batches of one kind stay within.
 struct PinnedWords {                                   // four int32 words the device writes and the host polls
     std::mutex mutex;
     std::vector<at::Tensor> free;
@@ -148,19 +149,21 @@ PinnedWords& pinned_words() {
     return *pool;
 }
 
-struct EdgeHints {                                     // edge count of the last search of a shape
+struct EdgeHints {                                     // largest recent edge count of a shape: falls by an eighth of the way
     using Key = std::tuple<int, int, float, float, float, float>;
     std::mutex mutex;
     std::map<Key, int> counts;
-    int64_t get(const Key& k, int64_t otherwise) {
+    // capacity for the next search, given the count of a uniform system
+    int64_t capacity(const Key& k, double uniform) {
         std::lock_guard<std::mutex> lock(mutex);
         auto it = counts.find(k);
-        return it == counts.end() ? otherwise : it->second;
+        return 1024 + (int64_t)(it == counts.end() ? 1.125 * std::min(uniform, 1.9e9) : 1.025 * it->second);
     }
     void put(const Key& k, int n) {
         std::lock_guard<std::mutex> lock(mutex);
         if (counts.size() > 256) counts.clear();
-        counts[k] = n;
+        int& kept = counts.emplace(k, n).first->second;
+        kept = std::max(n, kept - (kept - n) / 8);
     }
 };
 EdgeHints& edge_hints() {
@@ -184,9 +187,8 @@ py::object radius_graph(int listmax, int neighboursmax, float cutoff, float bx, 
     const mg_stream_t stream = stream_of(x);
     check(mg_graph_search(fp(x), batch, nodes, cutoff, bx, by, bz, workspace.data_ptr(), bytes, stream));
     const EdgeHints::Key key{batch, nodes, cutoff, bx, by, bz};
-    const double mean = atoms > 0 ? 1.5 * atoms * (nodes / ((double)bx * by * bz)) * 4.18879 * cutoff * cutoff * cutoff : 0.0;
-    int64_t capacity = (int64_t)(1.125 * edge_hints().get(key, (int64_t)std::min(mean, 2e9))) + 4096;
-    capacity = std::min<int64_t>(capacity, 0x7fffffff);
+    const double uniform = atoms > 0 ? atoms * (nodes / ((double)bx * by * bz)) * 4.18879 * cutoff * cutoff * cutoff : 0.0;
+    int64_t capacity = std::min<int64_t>(edge_hints().capacity(key, uniform), 0x7fffffff);
     at::Tensor src, dst, src64, dst64, r_ij;
     at::Tensor words = pinned_words().take();
     volatile int* w = words.data_ptr<int>();
