@@ -16,6 +16,8 @@
 // channels, edge vectors not differentiated: 0.72 ms (5.8 TB/s) and 0.42 ms (4.2 TB/s).  Before, the filters were stored
 // (0.44 ms), two kernels gathered the 60 gradients at every edge's source (1.8 ms each), a third took the right operands'
 // gradients to enc and rh (0.35 ms) and three segment sums followed (0.37 ms).
+// Any multiple of 64 channels; differentiable.message_products comes here for multiples of 256, the widths of its forward
+// kernels, and keeps the plain formulation for others.
 // The per-edge gradients are stored rather than formed again by destination, which would gather the 60 floats of the source
 // for every edge instead of writing and reading 13.
 #include "common.hpp"

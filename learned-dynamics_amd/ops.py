@@ -1173,8 +1173,8 @@ def tensor_linear_fwd(inds, W, x, bias=None, act=ACT_NONE, out=None, accumulate=
     want_rowmax: return (y, rowmax) with rowmax ((GEMM rows), parts) partial row maxima of |y| when the kernel
     that ran can emit them (plain-row output through the split-fp16 path), else (y, None).
     x_rows: components_as_rows(inds, x) of this same x, if the caller has it (None is allowed).
-    sequential: the reduction of an element runs over k in order whatever the number of rows is (few rows otherwise
-    split it over the waves of a workgroup)."""
+    sequential: the reduction of an element runs over k in order (few rows otherwise split it over the waves of a
+    workgroup), in fp32 below 256 rows (32 768 rows x components), from the fp16 pieces above."""
     x2, x2max = x_rows if x_rows is not None else (None, None)
     y, ymax = _ext.linear_fwd(inds, W, x, bias, act, out, accumulate, x_layout, y_layout, *_bound_parts(row_bound),
                               rows_per_bound, want_rowmax, x2, x2max, sequential)

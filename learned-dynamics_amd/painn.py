@@ -218,8 +218,10 @@ class Message(nn.Module):
 
     use_sliced = True
     use_cell_order = True
-    # Edges from which the filter MLP's last layers run inside the edge kernel.  Its tiles are 256 edges x 256 columns: 6000
-    # edges are 47 workgroups and take 61 us, a stored filter from GEMMs cut to the problem and the plain edge kernel 25.
+    # Edges from which the filter MLP's last layers run inside the edge kernel, whose tiles of 256 edges x 256 columns leave CUs
+    # idle below.  The whole message, filter stored / folded, us, for (n, n_rbf): (64, 16) 82 / 94 at 8192 edges, 108 / 107 at
+    # 24 576, 116 / 113 at 32 768, 172 / 130 at 65 536; (128, 128) 114 / 129, 173 / 172, 214 / 203, 389 / 371; (128, 32) crosses
+    # at 24 576 too, (64, 64) at about 57 000 (112 / 121 at 32 768, 164 / 157 at 65 536).
     FOLD_EDGES = 32768
 
     def _sliced_actv_last(self):

@@ -26,10 +26,12 @@ class _TensorLinearFn(torch.autograd.Function):
     (archs/meanflow_painn8.py:274-282); the reference's C++ backward calls raw kernels and cannot.
     x_bound: row maxima of |x| when the caller already holds them (a scaling hint, not differentiated).
     bias (plain rows only): added in the kernel's epilogue; its gradient comes out of the weight-gradient pass.
-    sequential: every element's reduction in k order whatever the number of rows (ops.tensor_linear_fwd).  The layers that
-    lead to a LeakyReLU ask for it in their forward pass: the derivative jumps at zero, so a pre-activation within rounding
-    of zero takes one slope or the other, and a row's gradient must not depend on the size of the batch around it.
-    Gradients, and networks of smooth activations, take the faster split reduction."""
+    sequential: every element's reduction in k order, never split over the waves of a workgroup (ops.tensor_linear_fwd).  The
+    layers that lead to a LeakyReLU ask for it in their forward pass: the derivative jumps at zero, so a pre-activation within
+    rounding of zero takes one slope or the other, and these layers keep one kernel, and with it one order, for all sizes up to
+    a line (256 rows without components, 32 768 rows x components) and another above it.  Two batches on the same side of the
+    line give a row the same bits; across it, or against the same module under no_grad, which takes the split reduction, the
+    roundings differ.  Gradients, and networks of smooth activations, take the faster split reduction."""
 
     @staticmethod
     def forward(ctx, inds, W, x, x_bound=None, bias=None, want_bound=False, sequential=False):
