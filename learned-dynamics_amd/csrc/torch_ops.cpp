@@ -6,6 +6,7 @@
 
 #include <atomic>
 #include <climits>
+#include <limits>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -163,7 +164,8 @@ at::Tensor packed_weight(const at::Tensor& W, bool f16) {
 }
 
 // (max_o sum_i |W[o, i]|, max_o |bias[o]|): |act(x W^T + bias)| <= |x|max * first + second for |act(z)| <= |z|; read back
-// once per version of the parameters, both with one copy, other Python threads running meanwhile
+// once per version of the parameters, both with one copy, other Python threads running meanwhile.  Infinite where a parameter
+// is NaN: no bound, and the next layer goes in fp32
 std::pair<float, float> norms_of(const at::Tensor& W, const OptTensor& bias) {
     auto read = [](std::vector<at::Tensor> t) {
         const at::Tensor stacked = at::stack(t);
@@ -176,14 +178,16 @@ std::pair<float, float> norms_of(const at::Tensor& W, const OptTensor& bias) {
     at::NoGradGuard no_grad;
     auto of_weight = [&] { return W.detach().abs().sum(1).amax(); };
     auto of_bias = [&] { return bias->detach().abs().amax(); };
-    constexpr float kAbove = 1.0f + 1e-6f;                    // (the product with a row maximum must not round below the bound)
+    auto bound = [](float v) {                                // (a product with a row maximum must not round below the true one)
+        return v == v ? v * (1.0f + 1e-6f) : std::numeric_limits<float>::infinity();
+    };
     auto& kept = cache<float>();
     if (bias.has_value() && !kept.has(W, 3, 0) && !kept.has(*bias, 4, 0)) {
         const auto both = read({of_weight(), of_bias()});
-        return {kept.get(W, 3, 0, [&] { return both.first * kAbove; }), kept.get(*bias, 4, 0, [&] { return both.second * kAbove; })};
+        return {kept.get(W, 3, 0, [&] { return bound(both.first); }), kept.get(*bias, 4, 0, [&] { return bound(both.second); })};
     }
-    const float weight = kept.get(W, 3, 0, [&] { return read({of_weight()}).first * kAbove; });
-    return {weight, bias.has_value() ? kept.get(*bias, 4, 0, [&] { return read({of_bias()}).first * kAbove; }) : 0.f};
+    const float weight = kept.get(W, 3, 0, [&] { return bound(read({of_weight()}).first); });
+    return {weight, bias.has_value() ? kept.get(*bias, 4, 0, [&] { return bound(read({of_bias()}).first); }) : 0.f};
 }
 
 // ------------------------------------------------------------------ linear maps
@@ -193,6 +197,12 @@ struct Bound {
     float mul = 1.f, add = 0.f;
     int64_t rows_per = 1;
 };
+
+// the bound behind a layer with these norms (infinite factors stay numbers: 0 * inf would be none)
+Bound through(const Bound& b, const std::pair<float, float>& norms) {
+    auto product = [](float x, float y) { return x == 0.f || y == 0.f ? 0.f : x * y; };
+    return Bound{b.base, product(b.mul, norms.first), product(b.add, norms.first) + norms.second, b.rows_per};
+}
 
 bool f16x2_takes(int64_t rows, int64_t dim_in, int64_t dim_out, const at::Tensor& x) {
     return dim_in % 32 == 0 && dim_in >= 64 && dim_out >= 8 && rows >= 1 && aligned16(x);
@@ -494,11 +504,7 @@ at::Tensor chain(at::Tensor h, const Tensors& W, const Tensors& b, const std::ve
             y = std::get<0>(linear_fwd(0, W[k], h, bias, act[k], OptTensor(y), false, 0, 0, OptTensor(), 1, 0, 1, false,
                                        OptTensor(), OptTensor(), false));
         }
-        if (bound.base.has_value() && k + 1 < W.size()) {
-            const auto [l1, bmax] = norms_of(W[k], bias);
-            bound.mul *= l1;
-            bound.add = bound.add * l1 + bmax;
-        }
+        if (bound.base.has_value() && k + 1 < W.size()) bound = through(bound, norms_of(W[k], bias));
         h = y;
     }
     return h;

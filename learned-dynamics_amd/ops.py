@@ -1090,6 +1090,7 @@ def linear_out_bound_factors(W, bias):
         with derived_tensors():
             both = torch.stack([W.detach().abs().sum(dim=1).amax(),
                                 bias.detach().abs().amax() if bias is not None else W.new_zeros(())]).tolist()
+        both = [float("inf") if v != v else v for v in both]           # (a NaN parameter: no bound)
         # a little above the float32 value: the product with a row maximum must not round below the true bound
         hit = (weakref.ref(W), w_ver, weakref.ref(bias) if bias is not None else None, b_ver,
                both[0] * (1.0 + 1e-6), both[1] * (1.0 + 1e-6))
@@ -1114,7 +1115,7 @@ class ScaledBound:
 
     def through(self, l1, bmax):
         """The bound after a linear layer with these norms (and any act with |act(z)| <= |z|)."""
-        return ScaledBound(self.base, self.mul * l1, self.add * l1 + bmax)
+        return ScaledBound(self.base, self.mul * l1 if self.mul else 0.0, (self.add * l1 if self.add else 0.0) + bmax)
 
     def tensor(self):
         b = self.base if self.base.size(1) == 1 else self.base.amax(dim=1, keepdim=True)
