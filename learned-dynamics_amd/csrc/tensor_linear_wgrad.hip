@@ -361,8 +361,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
             const long last_live = bias_rows - first_row(r) - 8 * octet;           // rows u < last_live have a bias
 #pragma unroll
             for (int u = 0; u < 8; u++) {
-                const float w = (u >= first_live && u < last_live && r < r_hi) ? 1.f : 0.f;
-                colsum.x += w * v[u].x; colsum.y += w * v[u].y; colsum.z += w * v[u].z; colsum.w += w * v[u].w;
+                const bool counts = u >= first_live && u < last_live && r < r_hi;  // (selected: 0 * inf would be NaN)
+                colsum.x += counts ? v[u].x : 0.f; colsum.y += counts ? v[u].y : 0.f;
+                colsum.z += counts ? v[u].z : 0.f; colsum.w += counts ? v[u].w : 0.f;
             }
         }
 #pragma unroll
