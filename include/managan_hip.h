@@ -369,6 +369,36 @@ typedef struct mg_f16x2_linear {
 } mg_f16x2_linear;
 int mg_tensor_linear_f16x2_run(const mg_f16x2_linear* args /* host */, mg_stream_t stream);
 int mg_tensor_linear_f16x2_rowmax_parts_sequential(long rows, int dim_in, int dim_out);
+/* Linear, SiLU, Linear, SiLU, Linear (archs/meanflow_painn8.py:38-51) on plain rows as one kernel, the hidden rows staying on
+ * chip: x (rows, dim_in) -> y (rows, dim), hidden layers of `dim` columns, packed_W from mg_linear_f16x2_pack_weight, biases
+ * of dim floats or NULL.  mg_mlp_f16x2_supported: multiples of 32 from 32 to 512.
+ * For the adjoint the forward call keeps, per hidden layer, z (its activation's input), h = SiLU(z) and the row maxima of |h| (all
+ * of them or none; x_rowmax, the row maxima of |x|, may be NULL by itself).  dual != 0: every array holds `rows` rows of values and
+ * then `rows` rows of forward-mode tangents, the biases apply to the values, and the adjoint is that of both.
+ * Adjoint: dy (rows, dim) -> dz of the two hidden layers with their row maxima, and dx (rows, dim_in) unless NULL;
+ * packed_Wt: the packed transposes of the weights (packed_Wt[0] may be NULL with dx).  Arrays are 16-byte aligned. */
+typedef struct mg_mlp_f16x2 {
+    const float* x;
+    long rows;
+    int dual, dim_in, dim;
+    const void* packed_W[3];
+    const float* bias[3];
+    float* y;
+    float *z[2], *h[2], *h_rowmax[2];
+    float* x_rowmax;
+} mg_mlp_f16x2;
+typedef struct mg_mlp_f16x2_grad {
+    const float* dy;
+    long rows;
+    int dual, dim_in, dim;
+    const void* packed_Wt[3];
+    const float* z[2];
+    float *dz[2], *dz_rowmax[2];
+    float* dx;
+} mg_mlp_f16x2_grad;
+int mg_mlp_f16x2_supported(int dim_in, int dim);      /* returns 0 / 1, not a status */
+int mg_mlp_f16x2_forward(const mg_mlp_f16x2* args /* host */, mg_stream_t stream);
+int mg_mlp_f16x2_adjoint(const mg_mlp_f16x2_grad* args /* host */, mg_stream_t stream);
 /* y = act(x W^T + bias) in float64 arithmetic: W (dim_out, dim_in) and bias are the float32 parameters, widened
  * exactly; x (rows, dim_in), every product and sum, the activation and y (rows, dim_out) are double.  The same
  * contraction as nn.Linear inside the reference's MLPs (archs/meanflow_painn8.py:38-51); float64 has no counterpart

@@ -125,6 +125,9 @@ _SIGNATURES = {
     "mg_bee_message_grad_run": [vp, vp],
     "mg_sort_by_key_workspace_bytes": [i64, vp],
     "mg_sort_by_key": [vp, i64, i32, vp, vp, vp, vp],
+    "mg_mlp_f16x2_supported": [i32, i32],
+    "mg_mlp_f16x2_forward": [vp, vp],
+    "mg_mlp_f16x2_adjoint": [vp, vp],
     "mg_silu_rows_fwd": [vp, i64, i32, i32, vp, vp, vp],
     "mg_silu_rows_bwd": [vp, vp, i64, i32, i32, vp, vp, vp],
     "mg_painn_edge_encode_fwd": [vp, vp, i64, i32, f32, f32, vp, vp, vp, vp, vp],

@@ -1,0 +1,496 @@
+// Linear, SiLU, Linear, SiLU, Linear on node- and edge-sized arrays of rows as one kernel, forward and adjoint, in the
+// split-fp16 arithmetic of f16x2.hpp.
+//
+// A workgroup takes 32 MI rows through all layers.  Their activations stay in LDS as fp16 pieces, in the order the matrix cores
+// read them; wave w owns the output columns [32 w, + 32) of every layer and reads the fragments of its part of the packed
+// weight straight from memory (one contiguous kilobyte per load, resident in the L2).  No barrier stands in
+// the loop over k; two stand between layers.  The weight is the A operand of v_mfma_f32_32x32x16_f16 and the rows are B, so
+// that a lane of the product holds 16 columns of ONE row in groups of four: bias and activation need no exchange, a row's
+// maximum takes one shuffle and a line of LDS, and the next layer's pieces are written eight bytes at a time, whole
+// rows being known to the workgroup: a layer's operand is scaled by its rows' own maxima.
+//
+// Layer by layer (three launches of linear_rows_f16x2_kernel) the same work writes and reads the hidden rows through memory, splits
+// a row once per column tile and carries bounds instead of maxima: 128 -> 512 -> 512 -> 512 on 16 336 rows 98 us there, 69 us
+// here, 4096 rows 62 and 34 us; 256 -> 384 87 and 52 us; 64 -> 256 53 and 26 us.  What bounds it: with 64 rows a workgroup the matrix cores are
+// busy for 25 of 40 thousand cycles of a 512 x 512 layer (sixteen waves issue in turn, waiting for fragments that 32 KB per step
+// and CU of L1 traffic delay), and 8 thousand go to activation, split and the two barriers; in long runs the board's power
+// (1.1 PFLOP/s for this mix of loads and products on its own, 0.9 here).  Eight waves with two column blocks each were slower
+// everywhere (78 us, 40 us): fewer waves to wait beside.
+#include "common.hpp"
+#include "f16x2.hpp"
+#include "silu.hpp"
+
+namespace mg {
+namespace {
+
+enum { kInfer = 0, kTrain = 1, kAdjoint = 2 };
+
+constexpr int kMaxDim = 512;       // widest layer: 64 rows of it are 128 KB of pieces
+constexpr int kMaxWaves = 16;
+
+struct MlpArgs {
+    const float* x;
+    long R;                        // rows of values; as many rows of tangents lie behind them in the dual kernels
+    int K, O, N;                   // columns of x, of the hidden layers, of y
+    const _Float16* planes[3];
+    const float* inv[3];           // inverse scales of the weights' rows, marks behind them
+    const float* bias[3];
+    float* y;
+    const float* z_in[2];          // adjoint: the hidden layers' inputs of their activation, in the order they are met
+    float *z[2], *h[2], *h_max[2]; // training: kept for the adjoint; adjoint: h, h_max are the gradients of z and their row maxima
+    float* x_max;
+};
+
+__device__ __forceinline__ int pad256(int o) { return (o + 255) / 256 * 256; }
+__device__ __forceinline__ bool has_marks(const float* inv, int O, int lane) {
+    const int* marks = reinterpret_cast<const int*>(inv + pad256(O));
+    return __any(lane < (O + 31) / 32 && marks[lane < (O + 31) / 32 ? lane : 0] != 0);
+}
+
+// acc[mi] = rows (pieces in LDS, xh at the first row block, mi_stride halves between them, lo pieces x_lo halves further on) times
+// the 32 weight rows whose fragments start at wp.  The two small products of a step have an accumulator of their own, and with
+// one row block the large ones have two: the large sum is rounded once per 16 or 32 k instead of three times per 16.
+template <int MI>
+__device__ __forceinline__ void multiply(const _Float16* __restrict__ wp, long w_lo, int K, const _Float16* xh, int mi_stride,
+                                         int x_lo, int lane, floatx16 (&acc)[MI]) {
+    constexpr int kSums = MI == 1 ? 2 : 1, kX = MI == 1 ? 2 : 1;   // (what 128 registers hold)
+    const int steps = K >> 4;                                      // (even)
+    const unsigned at = lane * 8;
+    xh += at;
+    halfx8 wh[2], wl[2], bh[kX][MI], bl[kX][MI];
+    floatx16 large[kSums][MI], small[MI];
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            small[mi][q] = 0.f;
+#pragma unroll
+            for (int k = 0; k < kSums; k++) large[k][mi][q] = 0.f;
+        }
+    auto load_w = [&](int u, int s) {
+        const _Float16* p = wp + 512L * (s < steps ? s : steps - 1);      // (surplus loads of the last trip are never used)
+        wh[u] = *reinterpret_cast<const halfx8*>(p + at);
+        wl[u] = *reinterpret_cast<const halfx8*>(p + w_lo + at);
+    };
+    auto load_x = [&](int u, int s) {
+        const int off = 512 * (s < steps ? s : steps - 1);
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++) {
+            bh[u][mi] = *reinterpret_cast<const halfx8*>(xh + mi * mi_stride + off);
+            bl[u][mi] = *reinterpret_cast<const halfx8*>(xh + x_lo + mi * mi_stride + off);
+        }
+    };
+    load_w(0, 0);
+    load_w(1, 1);
+    if (kX == 2) load_x(0, 0);
+    for (int s = 0; s < steps; s += 2) {                           // (no branch inside: the loads stay in flight across trips)
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int x = kX == 2 ? u : 0;
+            __builtin_amdgcn_sched_barrier(0);                     // keep this issue order
+            load_x(kX == 2 ? 1 - u : 0, kX == 2 ? s + u + 1 : s + u);
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++) {
+                small[mi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wh[u], bl[x][mi], small[mi], 0, 0, 0);
+                large[u % kSums][mi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wh[u], bh[x][mi], large[u % kSums][mi], 0, 0, 0);
+            }
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++) small[mi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wl[u], bh[x][mi], small[mi], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            load_w(u, s + u + 2);
+        }
+    }
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++) {
+        acc[mi] = small[mi] + large[0][mi];
+        if (kSums == 2) acc[mi] += large[kSums - 1][mi];
+    }
+}
+
+// Where k of a row lies among the pieces of its row block: step, lane of the fragment, k & 7
+__device__ __forceinline__ int piece_at(int row, int k) {
+    return (((k >> 5) * 2 + ((k >> 3) & 1)) * 64 + row + 32 * ((k >> 4) & 1)) * 8 + (k & 7);
+}
+
+// four consecutive k of a row as pieces, or the bits of the fp32 values where the pieces cannot carry the row
+__device__ __forceinline__ void store_pieces(_Float16* xh, int x_lo, int at, const float (&v)[4], float scale) {
+    halfx4 hi, lo;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float x = v[i] * scale;
+        const _Float16 h = (_Float16)x;
+        hi[i] = h;
+        lo[i] = (_Float16)(x - (float)h);
+    }
+    *reinterpret_cast<halfx4*>(xh + at) = hi;
+    *reinterpret_cast<halfx4*>(xh + x_lo + at) = lo;
+}
+__device__ __forceinline__ void store_bits(_Float16* xh, int x_lo, int at, const float (&v)[4]) {
+    ushort4 hi, lo;
+    const unsigned b[4] = {__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
+    hi = make_ushort4(b[0] >> 16, b[1] >> 16, b[2] >> 16, b[3] >> 16);
+    lo = make_ushort4(b[0] & 0xffff, b[1] & 0xffff, b[2] & 0xffff, b[3] & 0xffff);
+    *reinterpret_cast<ushort4*>(xh + at) = hi;
+    *reinterpret_cast<ushort4*>(xh + x_lo + at) = lo;
+}
+
+// x . w in fp32, k in order, for a row that lies in LDS as bits; weight row n put together from its pieces (row_in_fp32)
+__device__ __noinline__ float lds_row_in_fp32(const _Float16* xh, int x_lo, int row, const _Float16* planes, long plane_elems, long n,
+                                              int K, float iw) {
+    const float inv = unmark_weight(iw);
+    float sum = 0.f;
+#pragma unroll 1
+    for (int k = 0; k < K; k += 8) {
+        const int xa = piece_at(row, k);
+        const long at = packed_index(n, k, K);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const unsigned hi = __builtin_bit_cast(unsigned short, xh[xa + j]), lo = __builtin_bit_cast(unsigned short, xh[x_lo + xa + j]);
+            const float h = (float)planes[at + j], l = (float)planes[plane_elems + at + j];
+            sum = fmaf(__uint_as_float(hi << 16 | lo), (fabsf(h) < __builtin_inff() ? h + l : h) * inv, sum);
+        }
+    }
+    return sum;
+}
+
+template <int MI, int MODE, bool DUAL>
+__global__ void __launch_bounds__(64 * kMaxWaves) mlp_f16x2_kernel(const MlpArgs a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    static_assert(!DUAL || MI == 2, "values and tangents are the two row blocks");
+    constexpr int TM = 32 * MI;
+    const int O = a.O, widest = a.K > O ? a.K : O;
+    _Float16* const xh = reinterpret_cast<_Float16*>(lds);
+    float* const row_max = reinterpret_cast<float*>(lds + (size_t)TM * widest * 4);      // [waves][TM]
+    float* const fixed = row_max + kMaxWaves * TM;                                       // [kMaxDim]
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
+    const int m = lane & 31, G = lane >> 5;
+    const long r0 = (long)blockIdx.x * (DUAL ? 32 : TM);
+    // rows past the end repeat the last one and are not written
+    auto row_of = [&](int mi, int mm) { const long r = r0 + (DUAL ? 0 : 32 * mi) + mm; return (r < a.R ? r : a.R - 1) + (DUAL ? mi * a.R : 0); };
+    auto live = [&](int mi) { return r0 + (DUAL ? 0 : 32 * mi) + m < a.R; };
+
+    float isx[MI];
+    bool odd[MI];
+    {   // the rows of x: eight lanes to a row, whole rows in registers between the maximum and the split
+        const int K = a.K, x_lo = TM * K, p = lane & 7;
+        const bool marked = has_marks(a.inv[0], a.O, lane);
+        for (int grp = wave; grp < 4 * MI; grp += waves) {
+            const int lr = grp * 8 + (lane >> 3), mi = lr >> 5, mm = lr & 31;
+            const float* row = a.x + row_of(mi, mm) * K + 4 * p;
+            float v[kMaxDim / 32][4];
+            float mx = 0.f;
+#pragma unroll
+            for (int j = 0; j < kMaxDim / 32; j++)
+                if (32 * j < K) {
+                    const float4 f = *reinterpret_cast<const float4*>(row + 32 * j);
+                    v[j][0] = f.x; v[j][1] = f.y; v[j][2] = f.z; v[j][3] = f.w;
+                }
+#pragma unroll
+            for (int j = 0; j < kMaxDim / 32; j++)
+                if (32 * j < K)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) mx = fmaxf(mx, fabsf(v[j][i]));
+#pragma unroll
+            for (int d = 1; d < 8; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
+            float inv;
+            const float scale = pow2_scale(mx, &inv);
+            const bool bits = marked || beyond_split(mx);
+            const int at = mi * 32 * K + piece_at(mm, 4 * p);
+#pragma unroll
+            for (int j = 0; j < kMaxDim / 32; j++)
+                if (32 * j < K) store_pieces(xh, x_lo, at + 1024 * j, v[j], scale);
+            if (__any(bits))                                       // (rare)
+#pragma unroll
+                for (int j = 0; j < kMaxDim / 32; j++)
+                    if (32 * j < K && bits) store_bits(xh, x_lo, at + 1024 * j, v[j]);
+            if (p == 0) row_max[lr] = mx;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++) {
+            const float mx = row_max[32 * mi + m];
+            pow2_scale(mx, &isx[mi]);
+            odd[mi] = marked || beyond_split(mx);
+            if (MODE == kTrain && a.x_max && wave == 0 && G == 0 && live(mi)) a.x_max[row_of(mi, m)] = mx;
+        }
+        __syncthreads();                                           // (row_max is written again below)
+    }
+
+    constexpr int kFull = MODE == kAdjoint ? 2 : 3;                // layers with O columns
+    int K = a.K;
+#pragma unroll 1
+    for (int l = 0; l < kFull; l++) {
+        const int x_lo = TM * K;
+        const long w_lo = (long)pad256(O) * K;
+        const float* inv = a.inv[l];
+        floatx16 acc[MI];
+        multiply<MI>(a.planes[l] + (long)wave * (K >> 5) * 1024, w_lo, K, xh, 32 * K, x_lo, lane, acc);
+
+        // rows that the pieces cannot carry (all waves see the same ones)
+        bool any_odd = false;
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++) any_odd |= __any(odd[mi]);
+        if (any_odd) {
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++) {
+                unsigned rows = (unsigned)__ballot(odd[mi]);
+                while (rows) {
+                    const int r = __builtin_ctz(rows);
+                    rows &= rows - 1;
+                    if (tid < O) fixed[tid] = lds_row_in_fp32(xh + mi * 32 * K, x_lo, r, a.planes[l], w_lo, tid, K, inv[tid]);
+                    __syncthreads();
+#pragma unroll
+                    for (int q = 0; q < 16; q++) {
+                        const float f = fixed[32 * wave + 8 * (q / 4) + 4 * G + q % 4];
+                        if (m == r) acc[mi][q] = f;
+                    }
+                    __syncthreads();
+                }
+            }
+        }
+
+        const bool last = MODE != kAdjoint && l == kFull - 1;
+        float mx[MI];
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++) mx[mi] = 0.f;
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const int col = 32 * wave + 8 * t + 4 * G;
+                const float4 iw4 = *reinterpret_cast<const float4*>(inv + col);
+                const float iw[4] = {iw4.x, iw4.y, iw4.z, iw4.w};
+                float b[4] = {0.f, 0.f, 0.f, 0.f};
+                if constexpr (MODE != kAdjoint)
+                    if (a.bias[l]) {
+                        const float4 b4 = *reinterpret_cast<const float4*>(a.bias[l] + col);
+                        b[0] = b4.x; b[1] = b4.y; b[2] = b4.z; b[3] = b4.w;
+                    }
+                float v[MI][4];
+#pragma unroll
+                for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const float p = acc[mi][4 * t + i];
+                        v[mi][i] = (odd[mi] ? p : p * isx[mi] * iw[i]) + (DUAL && mi == 1 ? 0.f : b[i]);
+                    }
+                auto put = [&](float* dst, int mi, const float (&w)[4]) {
+                    if (live(mi)) *reinterpret_cast<float4*>(dst + row_of(mi, m) * O + col) = make_float4(w[0], w[1], w[2], w[3]);
+                };
+                if (last) {
+#pragma unroll
+                    for (int mi = 0; mi < MI; mi++) put(a.y, mi, v[mi]);
+                    continue;
+                }
+                if constexpr (MODE == kInfer) {
+#pragma unroll
+                    for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) v[mi][i] = v[mi][i] * __builtin_amdgcn_rcpf(1.0f + __expf(-v[mi][i]));
+                } else if constexpr (MODE == kTrain) {
+#pragma unroll
+                    for (int mi = 0; mi < MI; mi++) put(a.z[l], mi, v[mi]);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const Silu s = silu(v[0][i]);
+                        v[0][i] = s.f;
+                        if constexpr (MI == 2) v[1][i] = DUAL ? s.d1 * v[1][i] : silu(v[1][i]).f;
+                    }
+#pragma unroll
+                    for (int mi = 0; mi < MI; mi++) put(a.h[l], mi, v[mi]);
+                } else {
+                    float4 z[MI];
+#pragma unroll
+                    for (int mi = 0; mi < MI; mi++) z[mi] = *reinterpret_cast<const float4*>(a.z_in[l] + row_of(mi, m) * O + col);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const float z0 = i == 0 ? z[0].x : i == 1 ? z[0].y : i == 2 ? z[0].z : z[0].w;
+                        const Silu s = silu(z0);
+                        v[0][i] *= s.d1;
+                        if constexpr (MI == 2) {
+                            const float z1 = i == 0 ? z[MI - 1].x : i == 1 ? z[MI - 1].y : i == 2 ? z[MI - 1].z : z[MI - 1].w;
+                            if constexpr (DUAL) {
+                                v[0][i] += v[1][i] * z1 * s.d2;
+                                v[1][i] *= s.d1;
+                            } else {
+                                v[1][i] *= silu(z1).d1;
+                            }
+                        }
+                    }
+#pragma unroll
+                    for (int mi = 0; mi < MI; mi++) put(a.h[l], mi, v[mi]);
+                }
+#pragma unroll
+                for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        acc[mi][4 * t + i] = v[mi][i];
+                        mx[mi] = fmaxf(mx[mi], fabsf(v[mi][i]));
+                    }
+            }
+        if (last) return;
+
+        // the next layer's rows: their maxima, then their pieces in the place of this layer's
+        const bool marked = has_marks(a.inv[l + 1 < kFull ? l + 1 : kFull - 1], O, lane) ||
+                            (MODE == kAdjoint && l + 1 == kFull && a.y && has_marks(a.inv[2], a.N, lane));
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++) {
+            mx[mi] = fmaxf(mx[mi], __shfl_xor(mx[mi], 32));
+            if (G == 0) row_max[wave * TM + 32 * mi + m] = mx[mi];
+        }
+        __syncthreads();
+        K = O;
+        const int lo = TM * O;
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++) {
+            float top = 0.f;
+            for (int w = 0; w < waves; w++) top = fmaxf(top, row_max[w * TM + 32 * mi + m]);
+            const float scale = pow2_scale(top, &isx[mi]);
+            odd[mi] = marked || beyond_split(top);
+            if (MODE != kInfer && wave == 0 && G == 0 && live(mi)) a.h_max[l][row_of(mi, m)] = top;
+            auto each = [&](auto store) {
+#pragma unroll
+                    for (int t = 0; t < 4; t++) {
+                        const float v[4] = {acc[mi][4 * t], acc[mi][4 * t + 1], acc[mi][4 * t + 2], acc[mi][4 * t + 3]};
+                        store(mi * 32 * O + piece_at(m, 32 * wave + 8 * t + 4 * G), v);
+                    }
+            };
+            each([&](int at, const float (&v)[4]) { store_pieces(xh, lo, at, v, scale); });
+            if (__any(odd[mi]))                                    // (rare)
+                each([&](int at, const float (&v)[4]) { if (odd[mi]) store_bits(xh, lo, at, v); });
+        }
+        __syncthreads();
+    }
+
+    // adjoint: the gradient of x, O -> N columns, in units of 32 rows x 32 columns
+    if constexpr (MODE == kAdjoint) {
+        if (!a.y) return;
+        const int N = a.N, x_lo = TM * O, units = MI * (N / 32);
+        const long w_lo = (long)pad256(N) * O;
+        const float* inv = a.inv[2];
+#pragma unroll 1
+        for (int u = wave; u < units; u += waves) {
+            const int mi = MI == 1 ? 0 : u & 1, nb = u / MI;
+            floatx16 acc[1];
+            multiply<1>(a.planes[2] + (long)nb * (O >> 5) * 1024, w_lo, O, xh + mi * 32 * O, 0, x_lo, lane, acc);
+            const bool row_odd = mi == 0 ? odd[0] : odd[MI - 1];
+            const float row_isx = mi == 0 ? isx[0] : isx[MI - 1];
+            if (!live(mi)) continue;
+            float* out = a.y + row_of(mi, m) * N + 32 * nb + 4 * G;
+            if (row_odd) {
+#pragma unroll 1
+                for (int q = 0; q < 16; q++) {
+                    const int c = 8 * (q / 4) + q % 4;
+                    out[c] = lds_row_in_fp32(xh + mi * 32 * O, x_lo, m, a.planes[2], w_lo, 32 * nb + 4 * G + c, O, inv[32 * nb + 4 * G + c]);
+                }
+                continue;
+            }
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const float4 iw = *reinterpret_cast<const float4*>(inv + 32 * nb + 8 * t + 4 * G);
+                *reinterpret_cast<float4*>(out + 8 * t) =
+                    make_float4(acc[0][4 * t] * row_isx * iw.x, acc[0][4 * t + 1] * row_isx * iw.y,
+                                acc[0][4 * t + 2] * row_isx * iw.z, acc[0][4 * t + 3] * row_isx * iw.w);
+            }
+        }
+    }
+}
+
+template <int MI, int MODE, bool DUAL>
+int launch(const MlpArgs& a, hipStream_t st) {
+    const auto kernel = mlp_f16x2_kernel<MI, MODE, DUAL>;
+    const int widest = a.K > a.O ? a.K : a.O;
+    const size_t lds = (size_t)32 * MI * widest * 4 + (kMaxWaves * 32 * MI + kMaxDim) * sizeof(float);
+    // more than 64 KB of dynamic LDS has to be asked for (per device, so on every call)
+    if (lds > 65536) MG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const long tiles = ceil_div(a.R, DUAL ? 32 : 32 * MI);
+    MG_REQUIRE(tiles <= 0x7fffffffL, "mg_mlp_f16x2: grid too large (rows=%ld)", a.R);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(2 * a.O), lds, st, a);
+    return check_launch("mg_mlp_f16x2");
+}
+
+template <int MODE>
+int choose(const MlpArgs& a, bool dual, hipStream_t st) {
+    if constexpr (MODE != kInfer)
+        if (dual) return launch<2, MODE, true>(a, st);
+    // 32 rows a workgroup while the chip holds all of them at once, 64 beyond (the weights are read half as often):
+    // 128 -> 512 on 8192 rows 42 against 53 us, on 16 336 83 against 69; 128 -> 128 on 16 336 14.5 against 18.0
+    const int mi = ceil_div(a.R, 32) * (a.O / 32) > 256 * kMaxWaves ? 2 : 1;
+    return mi == 2 ? launch<2, MODE, false>(a, st) : launch<1, MODE, false>(a, st);
+}
+
+int fill(MlpArgs& a, const void* const* packed, int K, int O, int N) {
+    for (int l = 0; l < 3; l++) {
+        // (forward: K -> O -> O -> O; adjoint: O -> O -> O -> N)
+        const int in = l == 0 ? K : O, out = l == 2 ? N : O;
+        if (!packed[l]) continue;
+        if (!aligned16(packed[l])) return 0;
+        a.planes[l] = static_cast<const _Float16*>(packed[l]);
+        a.inv[l] = reinterpret_cast<const float*>(a.planes[l] + 2L * ((out + 255) / 256 * 256) * in);
+    }
+    return 1;
+}
+
+}  // namespace
+}  // namespace mg
+
+using namespace mg;
+
+extern "C" {
+
+int mg_mlp_f16x2_supported(int dim_in, int dim) {
+    return dim_in >= 32 && dim_in <= kMaxDim && dim_in % 32 == 0 && dim >= 32 && dim <= kMaxDim && dim % 32 == 0;
+}
+
+int mg_mlp_f16x2_forward(const mg_mlp_f16x2* p, mg_stream_t stream) {
+    MG_REQUIRE(p != nullptr && p->rows >= 0 && mg_mlp_f16x2_supported(p->dim_in, p->dim),
+               "mg_mlp_f16x2_forward: dimensions must be multiples of 32 up to %d", kMaxDim);
+    if (p->rows == 0) return MG_OK;
+    MlpArgs a{};
+    a.x = p->x;
+    a.R = p->rows;
+    a.K = p->dim_in;
+    a.O = a.N = p->dim;
+    a.y = p->y;
+    a.x_max = p->x_rowmax;
+    bool keep = false, keep_all = true;
+    for (int l = 0; l < 2; l++) {
+        a.z[l] = p->z[l];
+        a.h[l] = p->h[l];
+        a.h_max[l] = p->h_rowmax[l];
+        keep |= p->z[l] || p->h[l] || p->h_rowmax[l];
+        keep_all &= p->z[l] && p->h[l] && p->h_rowmax[l] && aligned16(p->z[l]) && aligned16(p->h[l]);
+    }
+    for (int l = 0; l < 3; l++) {
+        a.bias[l] = p->bias[l];
+        MG_REQUIRE(p->packed_W[l] && (!p->bias[l] || aligned16(p->bias[l])), "mg_mlp_f16x2_forward: null or unaligned weight or bias");
+    }
+    MG_REQUIRE(fill(a, p->packed_W, a.K, a.O, a.N) && a.x && a.y && aligned16(a.x) && aligned16(a.y) && keep == (keep && keep_all) &&
+                   (keep || !p->dual),
+               "mg_mlp_f16x2_forward: null or unaligned pointer");
+    return keep ? choose<kTrain>(a, p->dual, (hipStream_t)stream) : choose<kInfer>(a, false, (hipStream_t)stream);
+}
+
+int mg_mlp_f16x2_adjoint(const mg_mlp_f16x2_grad* p, mg_stream_t stream) {
+    MG_REQUIRE(p != nullptr && p->rows >= 0 && mg_mlp_f16x2_supported(p->dim_in, p->dim),
+               "mg_mlp_f16x2_adjoint: dimensions must be multiples of 32 up to %d", kMaxDim);
+    if (p->rows == 0) return MG_OK;
+    MlpArgs a{};
+    a.x = p->dy;
+    a.R = p->rows;
+    a.K = a.O = p->dim;
+    a.N = p->dim_in;
+    a.y = p->dx;
+    for (int l = 0; l < 2; l++) {                                  // met in reverse
+        a.z_in[l] = p->z[1 - l];
+        a.h[l] = p->dz[1 - l];
+        a.h_max[l] = p->dz_rowmax[1 - l];
+        MG_REQUIRE(a.z_in[l] && a.h[l] && a.h_max[l] && aligned16(a.z_in[l]) && aligned16(a.h[l]),
+                   "mg_mlp_f16x2_adjoint: null or unaligned pointer");
+    }
+    const void* packed[3] = {p->packed_Wt[2], p->packed_Wt[1], p->packed_Wt[0]};
+    MG_REQUIRE(fill(a, packed, a.O, a.O, a.N) && packed[0] && packed[1] && (packed[2] || !a.y) && a.x && aligned16(a.x) && aligned16(a.y),
+               "mg_mlp_f16x2_adjoint: null or unaligned pointer");
+    return choose<kAdjoint>(a, p->dual, (hipStream_t)stream);
+}
+
+}  // extern "C"

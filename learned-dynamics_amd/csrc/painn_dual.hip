@@ -9,6 +9,7 @@
 // split-fp16 linears scale by come out of the pass that writes the rows.
 // DUAL = false: no tangents (R rows); the tangent operands are ignored.
 #include "common.hpp"
+#include "silu.hpp"
 #include <algorithm>
 
 namespace mg {
@@ -58,14 +59,6 @@ __device__ __forceinline__ Vec3x4 zero12() {
 #pragma unroll
     for (int q = 0; q < 12; q++) r.f[q] = 0.f;
     return r;
-}
-
-// SiLU and its first two derivatives: s = sigma(z), p = s (1 - s)
-struct Silu { float f, d1, d2; };
-__device__ __forceinline__ Silu silu(float z) {
-    const float s = 1.0f / (1.0f + expf(-z));
-    const float p = s * (1.0f - s);
-    return {z * s, s + z * p, p * (2.0f + z * (1.0f - 2.0f * s))};
 }
 
 // lanes that share a row of n values (n % 4 == 0): a power of two <= 64, so that a row never straddles waves

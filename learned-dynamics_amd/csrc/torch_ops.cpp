@@ -486,9 +486,47 @@ at::Tensor silu_order(const at::Tensor& z, int order, const OptTensor& mul) {
 // ------------------------------------------------------------------ MLPs (inference)
 using Tensors = std::vector<at::Tensor>;
 
+const std::vector<int> kSiluMlp{kActSilu, kActSilu, kActNone};
+
+// Whether the three layers of an MLP on x (rows, k) go through one kernel (k: W[0]'s columns after zero padding).
+// A workgroup reads all three weights whatever the number of rows, about 30 us of a kernel at 128 -> 512 -> 512 -> 512 and 10 us
+// at 128 -> 128: for wide layers of few rows the three launches that split the reduction of each over the chip are faster (us,
+// one kernel / three launches: 128 -> 512 29.9 / 18.9 at 337 rows, 30.6 / 26.5 at 1021, 31.2 / 33.2 at 1400, 33.7 / 61.8
+// at 4096, 69 / 98 at 16 336; 256 -> 384 23.2 / 22.9 at 1021, 25.1 / 43.2 at 4096; 64 -> 256 12.6 / 14.2 at 64 rows, 26 / 53
+// at 16 384; 128 -> 128 9.9 / 14.2 at 64).  Distance from float64 at 128 -> 512: 2.3e-7 against 2.2..2.5e-7 with split
+// reductions, 2.75e-7 against 4.1e-7 at 16 336 rows.
+constexpr int64_t kMlpWide = 256, kMlpWideRows = 1024;
+bool mlp_takes(int64_t rows, int64_t k, const Tensors& W, const Tensors& b, const at::Tensor& x) {
+    const int64_t dim = W[0].size(0);
+    if (mg_get_linear_mode() != kModeF16x2 || rows < (dim > kMlpWide ? kMlpWideRows : 1) || k < 64 || dim < 64 || !mg_mlp_f16x2_supported((int)k, (int)dim))
+        return false;
+    for (size_t l = 0; l < 3; l++)
+        if (W[l].size(0) != dim || (l > 0 && W[l].size(1) != dim) || !aligned16(b[l])) return false;
+    return aligned16(x);
+}
+
+at::Tensor mlp_fused(const at::Tensor& x, const Tensors& W, const Tensors& b) {
+    at::Tensor y = floats(x, {x.size(0), W[2].size(0)});
+    mg_mlp_f16x2 a{};
+    Tensors planes;                                           // (kept alive until the launch is queued)
+    for (int l = 0; l < 3; l++) {
+        planes.push_back(packed_f16x2(W[l], l == 0 ? x.size(1) : W[l].size(1)));
+        a.packed_W[l] = planes[l].data_ptr();
+        a.bias[l] = fp(b[l]);
+    }
+    a.x = fp(x);
+    a.rows = x.size(0);
+    a.dim_in = (int)x.size(1);
+    a.dim = (int)W[0].size(0);
+    a.y = fp(y);
+    check(mg_mlp_f16x2_forward(&a, stream_of(x)));
+    return y;
+}
+
 // a chain of linears with fused bias and activation; the row bounds the split-fp16 layers scale by travel as
 // mul * base + add through the layers' norms, so that only the first layer ever looks at the data for them
 at::Tensor chain(at::Tensor h, const Tensors& W, const Tensors& b, const std::vector<int>& act, Bound bound) {
+    if (act == kSiluMlp && mlp_takes(h.size(0), h.size(1), W, b, h)) return mlp_fused(h, W, b);
     for (size_t k = 0; k < W.size(); k++) {
         const int64_t rows = h.size(0), dim_in = W[k].size(1), dim_out = W[k].size(0);
         at::Tensor y = floats(h, {rows, dim_out});
@@ -530,8 +568,6 @@ at::Tensor linear_chain(const at::Tensor& x, const Tensors& W, const Tensors& b,
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     return chain(x, W, b, act, Bound{bound, (float)mul, (float)add});
 }
-
-const std::vector<int> kSiluMlp{kActSilu, kActSilu, kActNone};
 
 // ------------------------------------------------------------------ PaiNN layers (inference)
 // Update.forward: x_a (batch, nodes, n), x_v (batch, nodes, n, 3); W_lrv (3n, n) the stacked l, r, v maps
@@ -601,6 +637,7 @@ at::Tensor filter_grid(const at::Tensor& enc, const at::Tensor& unit, const Tens
     TORCH_CHECK(k > W[0].size(1) && k % 32 == 0 && mg_get_linear_mode() == kModeF16x2 && aligned16(enc),
                 "filter_grid: encodings of a wrong width");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(enc.device());
+    if (mlp_takes(rows, k, W, b, enc)) return mlp_fused(enc, W, b);
     at::Tensor h = floats(enc, {rows, W[0].size(0)});
     const OptTensor b0(b[0]);
     run_f16x2(W[0], k, fp(enc), rows, Bound{OptTensor(unit)}, b0, kActSilu, false, 1, h, nullptr, false);
