@@ -375,7 +375,7 @@ int mg_tensor_linear_f16x2_rowmax_parts_sequential(long rows, int dim_in, int di
  * For the adjoint the forward call keeps, per hidden layer, z (its activation's input), h = SiLU(z) and the row maxima of |h| (all
  * of them or none; x_rowmax, the row maxima of |x|, may be NULL by itself).  dual != 0: every array holds `rows` rows of values and
  * then `rows` rows of forward-mode tangents, the biases apply to the values, and the adjoint is that of both.
- * Adjoint: dy (rows, dim) -> dz of the two hidden layers with their row maxima, and dx (rows, dim_in) unless NULL;
+ * Adjoint: dy (rows, dim) -> dz of the two hidden layers with their row maxima, dx (rows, dim_in) and the row maxima of |dy| unless NULL;
  * packed_Wt: the packed transposes of the weights (packed_Wt[0] may be NULL with dx).  Arrays are 16-byte aligned. */
 typedef struct mg_mlp_f16x2 {
     const float* x;
@@ -395,6 +395,7 @@ typedef struct mg_mlp_f16x2_grad {
     const float* z[2];
     float *dz[2], *dz_rowmax[2];
     float* dx;
+    float* dy_rowmax;
 } mg_mlp_f16x2_grad;
 int mg_mlp_f16x2_supported(int dim_in, int dim);      /* returns 0 / 1, not a status */
 int mg_mlp_f16x2_forward(const mg_mlp_f16x2* args /* host */, mg_stream_t stream);

@@ -47,30 +47,36 @@ __device__ __forceinline__ bool has_marks(const float* inv, int O, int lane) {
     return __any(lane < (O + 31) / 32 && marks[lane < (O + 31) / 32 ? lane : 0] != 0);
 }
 
-// acc[mi] = rows (pieces in LDS, xh at the first row block, mi_stride halves between them, lo pieces x_lo halves further on) times
-// the 32 weight rows whose fragments start at wp.  The two small products of a step have an accumulator of their own, and with
-// one row block the large ones have two: the large sum is rounded once per 16 or 32 k instead of three times per 16.
-template <int MI>
+// acc[mi][ni] = rows (pieces in LDS, xh at the first row block, mi_stride halves between them, lo pieces x_lo halves further on)
+// times the 32 NI weight rows whose fragments start at wp.  The two small products of a step have an accumulator of their own, and
+// with SUMS = 2 the large ones have two: the large sum is rounded once per 16 or 32 k instead of three times per 16.
+template <int MI, int NI, int SUMS>
 __device__ __forceinline__ void multiply(const _Float16* __restrict__ wp, long w_lo, int K, const _Float16* xh, int mi_stride,
-                                         int x_lo, int lane, floatx16 (&acc)[MI]) {
-    constexpr int kSums = MI == 1 ? 2 : 1, kX = MI == 1 ? 2 : 1;   // (what 128 registers hold)
+                                         int x_lo, int lane, floatx16 (&acc)[MI][NI]) {
+    constexpr int kX = SUMS;                                       // (buffers of x: what the registers hold)
     const int steps = K >> 4;                                      // (even)
     const unsigned at = lane * 8;
+    const long ni_stride = (long)(K >> 5) * 1024;
     xh += at;
-    halfx8 wh[2], wl[2], bh[kX][MI], bl[kX][MI];
-    floatx16 large[kSums][MI], small[MI];
+    halfx8 wh[2][NI], wl[2][NI], bh[kX][MI], bl[kX][MI];
+    floatx16 large[SUMS][MI][NI], small[MI][NI];
 #pragma unroll
     for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-        for (int q = 0; q < 16; q++) {
-            small[mi][q] = 0.f;
+        for (int ni = 0; ni < NI; ni++)
 #pragma unroll
-            for (int k = 0; k < kSums; k++) large[k][mi][q] = 0.f;
-        }
+            for (int q = 0; q < 16; q++) {
+                small[mi][ni][q] = 0.f;
+#pragma unroll
+                for (int k = 0; k < SUMS; k++) large[k][mi][ni][q] = 0.f;
+            }
     auto load_w = [&](int u, int s) {
         const _Float16* p = wp + 512L * (s < steps ? s : steps - 1);      // (surplus loads of the last trip are never used)
-        wh[u] = *reinterpret_cast<const halfx8*>(p + at);
-        wl[u] = *reinterpret_cast<const halfx8*>(p + w_lo + at);
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++) {
+            wh[u][ni] = *reinterpret_cast<const halfx8*>(p + ni * ni_stride + at);
+            wl[u][ni] = *reinterpret_cast<const halfx8*>(p + w_lo + ni * ni_stride + at);
+        }
     };
     auto load_x = [&](int u, int s) {
         const int off = 512 * (s < steps ? s : steps - 1);
@@ -90,21 +96,28 @@ __device__ __forceinline__ void multiply(const _Float16* __restrict__ wp, long w
             __builtin_amdgcn_sched_barrier(0);                     // keep this issue order
             load_x(kX == 2 ? 1 - u : 0, kX == 2 ? s + u + 1 : s + u);
 #pragma unroll
-            for (int mi = 0; mi < MI; mi++) {
-                small[mi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wh[u], bl[x][mi], small[mi], 0, 0, 0);
-                large[u % kSums][mi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wh[u], bh[x][mi], large[u % kSums][mi], 0, 0, 0);
-            }
+            for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-            for (int mi = 0; mi < MI; mi++) small[mi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wl[u], bh[x][mi], small[mi], 0, 0, 0);
+                for (int ni = 0; ni < NI; ni++) {
+                    small[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wh[u][ni], bl[x][mi], small[mi][ni], 0, 0, 0);
+                    large[u % SUMS][mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wh[u][ni], bh[x][mi], large[u % SUMS][mi][ni], 0, 0, 0);
+                }
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                for (int ni = 0; ni < NI; ni++)
+                    small[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wl[u][ni], bh[x][mi], small[mi][ni], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
             load_w(u, s + u + 2);
         }
     }
 #pragma unroll
-    for (int mi = 0; mi < MI; mi++) {
-        acc[mi] = small[mi] + large[0][mi];
-        if (kSums == 2) acc[mi] += large[kSums - 1][mi];
-    }
+    for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++) {
+            acc[mi][ni] = small[mi][ni] + large[0][mi][ni];
+            if (SUMS == 2) acc[mi][ni] += large[SUMS - 1][mi][ni];
+        }
 }
 
 // Where k of a row lies among the pieces of its row block: step, lane of the fragment, k & 7
@@ -153,22 +166,35 @@ __device__ __noinline__ float lds_row_in_fp32(const _Float16* xh, int x_lo, int 
     return sum;
 }
 
-template <int MI, int MODE, bool DUAL>
-__global__ void __launch_bounds__(64 * kMaxWaves) mlp_f16x2_kernel(const MlpArgs a) {
+// lanes 16 .. 31 (48 .. 63) of a and lanes 0 .. 15 (32 .. 47) of b change places; done twice, all is as before
+__device__ __forceinline__ void swap_rows(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+
+// DUAL: the 32 rows of a block are 16 values and their 16 tangents
+template <int MI, int NI, int MODE, bool DUAL>
+__global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const MlpArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    static_assert(!DUAL || MI == 2, "values and tangents are the two row blocks");
-    constexpr int TM = 32 * MI;
+    static_assert(!DUAL || MI == 1, "one block of values and tangents");
+    constexpr int TM = 32 * MI, kRows = DUAL ? 16 : TM;
+    constexpr int kSums = MI * NI == 1 ? 2 : 1;                    // (what 128 registers hold)
     const int O = a.O, widest = a.K > O ? a.K : O;
     _Float16* const xh = reinterpret_cast<_Float16*>(lds);
     float* const row_max = reinterpret_cast<float*>(lds + (size_t)TM * widest * 4);      // [waves][TM]
-    float* const fixed = row_max + kMaxWaves * TM;                                       // [kMaxDim]
+    float* const fixed = row_max + kMaxWaves / NI * TM;                                  // [kMaxDim]
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
     const int m = lane & 31, G = lane >> 5;
-    const long r0 = (long)blockIdx.x * (DUAL ? 32 : TM);
+    const long r0 = (long)blockIdx.x * kRows;
+    const bool tangent = DUAL && m >= 16;
     // rows past the end repeat the last one and are not written
-    auto row_of = [&](int mi, int mm) { const long r = r0 + (DUAL ? 0 : 32 * mi) + mm; return (r < a.R ? r : a.R - 1) + (DUAL ? mi * a.R : 0); };
-    auto live = [&](int mi) { return r0 + (DUAL ? 0 : 32 * mi) + m < a.R; };
+    auto row_of = [&](int mi, int mm) {
+        const long r = r0 + (DUAL ? mm & 15 : 32 * mi + mm);
+        return (r < a.R ? r : a.R - 1) + (DUAL && mm >= 16 ? a.R : 0);
+    };
+    auto live = [&](int mi) { return r0 + (DUAL ? m & 15 : 32 * mi + m) < a.R; };
 
     float isx[MI];
     bool odd[MI];
@@ -212,7 +238,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves) mlp_f16x2_kernel(const MlpArgs
             const float mx = row_max[32 * mi + m];
             pow2_scale(mx, &isx[mi]);
             odd[mi] = marked || beyond_split(mx);
-            if (MODE == kTrain && a.x_max && wave == 0 && G == 0 && live(mi)) a.x_max[row_of(mi, m)] = mx;
+            if (MODE != kInfer && a.x_max && wave == 0 && G == 0 && live(mi)) a.x_max[row_of(mi, m)] = mx;
         }
         __syncthreads();                                           // (row_max is written again below)
     }
@@ -224,8 +250,8 @@ __global__ void __launch_bounds__(64 * kMaxWaves) mlp_f16x2_kernel(const MlpArgs
         const int x_lo = TM * K;
         const long w_lo = (long)pad256(O) * K;
         const float* inv = a.inv[l];
-        floatx16 acc[MI];
-        multiply<MI>(a.planes[l] + (long)wave * (K >> 5) * 1024, w_lo, K, xh, 32 * K, x_lo, lane, acc);
+        floatx16 acc[MI][NI];
+        multiply<MI, NI, kSums>(a.planes[l] + (long)(wave * NI) * (K >> 5) * 1024, w_lo, K, xh, 32 * K, x_lo, lane, acc);
 
         // rows that the pieces cannot carry (all waves see the same ones)
         bool any_odd = false;
@@ -238,13 +264,16 @@ __global__ void __launch_bounds__(64 * kMaxWaves) mlp_f16x2_kernel(const MlpArgs
                 while (rows) {
                     const int r = __builtin_ctz(rows);
                     rows &= rows - 1;
-                    if (tid < O) fixed[tid] = lds_row_in_fp32(xh + mi * 32 * K, x_lo, r, a.planes[l], w_lo, tid, K, inv[tid]);
+                    for (int n = tid; n < O; n += blockDim.x)
+                        fixed[n] = lds_row_in_fp32(xh + mi * 32 * K, x_lo, r, a.planes[l], w_lo, n, K, inv[n]);
                     __syncthreads();
 #pragma unroll
-                    for (int q = 0; q < 16; q++) {
-                        const float f = fixed[32 * wave + 8 * (q / 4) + 4 * G + q % 4];
-                        if (m == r) acc[mi][q] = f;
-                    }
+                    for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+                        for (int q = 0; q < 16; q++) {
+                            const float f = fixed[32 * (wave * NI + ni) + 8 * (q / 4) + 4 * G + q % 4];
+                            if (m == r) acc[mi][ni][q] = f;
+                        }
                     __syncthreads();
                 }
             }
@@ -255,77 +284,92 @@ __global__ void __launch_bounds__(64 * kMaxWaves) mlp_f16x2_kernel(const MlpArgs
 #pragma unroll
         for (int mi = 0; mi < MI; mi++) mx[mi] = 0.f;
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const int col = 32 * wave + 8 * t + 4 * G;
-                const float4 iw4 = *reinterpret_cast<const float4*>(inv + col);
-                const float iw[4] = {iw4.x, iw4.y, iw4.z, iw4.w};
-                float b[4] = {0.f, 0.f, 0.f, 0.f};
-                if constexpr (MODE != kAdjoint)
-                    if (a.bias[l]) {
-                        const float4 b4 = *reinterpret_cast<const float4*>(a.bias[l] + col);
-                        b[0] = b4.x; b[1] = b4.y; b[2] = b4.z; b[3] = b4.w;
-                    }
-                float v[MI][4];
+        for (int ni = 0; ni < NI; ni++)
 #pragma unroll
-                for (int mi = 0; mi < MI; mi++)
+            for (int half = 0; half < 2; half++) {                 // (columns in two groups of four, 16 apart)
+                const int col = 32 * (wave * NI + ni) + 8 * half + 4 * G;
+                float iw[2][4], b[2][4];
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float p = acc[mi][4 * t + i];
-                        v[mi][i] = (odd[mi] ? p : p * isx[mi] * iw[i]) + (DUAL && mi == 1 ? 0.f : b[i]);
-                    }
-                auto put = [&](float* dst, int mi, const float (&w)[4]) {
-                    if (live(mi)) *reinterpret_cast<float4*>(dst + row_of(mi, m) * O + col) = make_float4(w[0], w[1], w[2], w[3]);
-                };
-                if (last) {
-#pragma unroll
-                    for (int mi = 0; mi < MI; mi++) put(a.y, mi, v[mi]);
-                    continue;
+                for (int k = 0; k < 2; k++) {
+                    const float4 w4 = *reinterpret_cast<const float4*>(inv + col + 16 * k);
+                    iw[k][0] = w4.x; iw[k][1] = w4.y; iw[k][2] = w4.z; iw[k][3] = w4.w;
+                    float4 b4 = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (MODE != kAdjoint && a.bias[l] && !tangent) b4 = *reinterpret_cast<const float4*>(a.bias[l] + col + 16 * k);
+                    b[k][0] = b4.x; b[k][1] = b4.y; b[k][2] = b4.z; b[k][3] = b4.w;
                 }
-                if constexpr (MODE == kInfer) {
 #pragma unroll
-                    for (int mi = 0; mi < MI; mi++)
+                for (int mi = 0; mi < MI; mi++) {
+                    float v[2][4];
+                    const bool alive = live(mi);
+                    const long at = row_of(mi, m) * O + col;
 #pragma unroll
-                        for (int i = 0; i < 4; i++) v[mi][i] = v[mi][i] * __builtin_amdgcn_rcpf(1.0f + __expf(-v[mi][i]));
-                } else if constexpr (MODE == kTrain) {
+                    for (int k = 0; k < 2; k++)
 #pragma unroll
-                    for (int mi = 0; mi < MI; mi++) put(a.z[l], mi, v[mi]);
+                        for (int i = 0; i < 4; i++) {
+                            const float p = acc[mi][ni][8 * k + 4 * half + i];
+                            v[k][i] = (odd[mi] ? p : p * isx[mi] * iw[k][i]) + b[k][i];
+                        }
+                    auto put = [&](float* dst) {
+                        if (!alive) return;
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const Silu s = silu(v[0][i]);
-                        v[0][i] = s.f;
-                        if constexpr (MI == 2) v[1][i] = DUAL ? s.d1 * v[1][i] : silu(v[1][i]).f;
+                        for (int k = 0; k < 2; k++) *reinterpret_cast<float4*>(dst + at + 16 * k) = make_float4(v[k][0], v[k][1], v[k][2], v[k][3]);
+                    };
+                    if (last) {
+                        put(a.y);
+                        continue;
                     }
+                    if constexpr (MODE == kInfer) {
 #pragma unroll
-                    for (int mi = 0; mi < MI; mi++) put(a.h[l], mi, v[mi]);
-                } else {
-                    float4 z[MI];
+                        for (int k = 0; k < 2; k++)
 #pragma unroll
-                    for (int mi = 0; mi < MI; mi++) z[mi] = *reinterpret_cast<const float4*>(a.z_in[l] + row_of(mi, m) * O + col);
+                            for (int i = 0; i < 4; i++) v[k][i] = v[k][i] * __builtin_amdgcn_rcpf(1.0f + __expf(-v[k][i]));
+                    } else if constexpr (MODE == kTrain) {
+                        put(a.z[l]);
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float z0 = i == 0 ? z[0].x : i == 1 ? z[0].y : i == 2 ? z[0].z : z[0].w;
-                        const Silu s = silu(z0);
-                        v[0][i] *= s.d1;
-                        if constexpr (MI == 2) {
-                            const float z1 = i == 0 ? z[MI - 1].x : i == 1 ? z[MI - 1].y : i == 2 ? z[MI - 1].z : z[MI - 1].w;
-                            if constexpr (DUAL) {
-                                v[0][i] += v[1][i] * z1 * s.d2;
+                        for (int i = 0; i < 4; i++) {
+                            if constexpr (DUAL) {                  // this lane: value and tangent of one of the two columns
+                                swap_rows(v[0][i], v[1][i]);
+                                const Silu s = silu(v[0][i]);
+                                v[0][i] = s.f;
                                 v[1][i] *= s.d1;
+                                swap_rows(v[0][i], v[1][i]);
                             } else {
-                                v[1][i] *= silu(z1).d1;
+                                v[0][i] = silu(v[0][i]).f;
+                                v[1][i] = silu(v[1][i]).f;
                             }
                         }
+                        put(a.h[l]);
+                    } else {
+                        float z[2][4];
+#pragma unroll
+                        for (int k = 0; k < 2; k++) {
+                            const float4 z4 = *reinterpret_cast<const float4*>(a.z_in[l] + at + 16 * k);
+                            z[k][0] = z4.x; z[k][1] = z4.y; z[k][2] = z4.z; z[k][3] = z4.w;
+                        }
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            if constexpr (DUAL) {
+                                swap_rows(v[0][i], v[1][i]);
+                                swap_rows(z[0][i], z[1][i]);
+                                const Silu s = silu(z[0][i]);
+                                v[0][i] = v[0][i] * s.d1 + v[1][i] * z[1][i] * s.d2;
+                                v[1][i] *= s.d1;
+                                swap_rows(v[0][i], v[1][i]);
+                            } else {
+                                v[0][i] *= silu(z[0][i]).d1;
+                                v[1][i] *= silu(z[1][i]).d1;
+                            }
+                        }
+                        put(a.h[l]);
                     }
 #pragma unroll
-                    for (int mi = 0; mi < MI; mi++) put(a.h[l], mi, v[mi]);
+                    for (int k = 0; k < 2; k++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            acc[mi][ni][8 * k + 4 * half + i] = v[k][i];
+                            mx[mi] = fmaxf(mx[mi], fabsf(v[k][i]));
+                        }
                 }
-#pragma unroll
-                for (int mi = 0; mi < MI; mi++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        acc[mi][4 * t + i] = v[mi][i];
-                        mx[mi] = fmaxf(mx[mi], fabsf(v[mi][i]));
-                    }
             }
         if (last) return;
 
@@ -349,9 +393,11 @@ __global__ void __launch_bounds__(64 * kMaxWaves) mlp_f16x2_kernel(const MlpArgs
             if (MODE != kInfer && wave == 0 && G == 0 && live(mi)) a.h_max[l][row_of(mi, m)] = top;
             auto each = [&](auto store) {
 #pragma unroll
+                for (int ni = 0; ni < NI; ni++)
+#pragma unroll
                     for (int t = 0; t < 4; t++) {
-                        const float v[4] = {acc[mi][4 * t], acc[mi][4 * t + 1], acc[mi][4 * t + 2], acc[mi][4 * t + 3]};
-                        store(mi * 32 * O + piece_at(m, 32 * wave + 8 * t + 4 * G), v);
+                        const float v[4] = {acc[mi][ni][4 * t], acc[mi][ni][4 * t + 1], acc[mi][ni][4 * t + 2], acc[mi][ni][4 * t + 3]};
+                        store(mi * 32 * O + piece_at(m, 32 * (wave * NI + ni) + 8 * t + 4 * G), v);
                     }
             };
             each([&](int at, const float (&v)[4]) { store_pieces(xh, lo, at, v, scale); });
@@ -361,61 +407,69 @@ __global__ void __launch_bounds__(64 * kMaxWaves) mlp_f16x2_kernel(const MlpArgs
         __syncthreads();
     }
 
-    // adjoint: the gradient of x, O -> N columns, in units of 32 rows x 32 columns
+    // adjoint: the gradient of x, O -> N columns, 32 to a wave at a time
     if constexpr (MODE == kAdjoint) {
         if (!a.y) return;
-        const int N = a.N, x_lo = TM * O, units = MI * (N / 32);
+        const int N = a.N, x_lo = TM * O;
         const long w_lo = (long)pad256(N) * O;
         const float* inv = a.inv[2];
 #pragma unroll 1
-        for (int u = wave; u < units; u += waves) {
-            const int mi = MI == 1 ? 0 : u & 1, nb = u / MI;
-            floatx16 acc[1];
-            multiply<1>(a.planes[2] + (long)nb * (O >> 5) * 1024, w_lo, O, xh + mi * 32 * O, 0, x_lo, lane, acc);
-            const bool row_odd = mi == 0 ? odd[0] : odd[MI - 1];
-            const float row_isx = mi == 0 ? isx[0] : isx[MI - 1];
-            if (!live(mi)) continue;
-            float* out = a.y + row_of(mi, m) * N + 32 * nb + 4 * G;
-            if (row_odd) {
-#pragma unroll 1
-                for (int q = 0; q < 16; q++) {
-                    const int c = 8 * (q / 4) + q % 4;
-                    out[c] = lds_row_in_fp32(xh + mi * 32 * O, x_lo, m, a.planes[2], w_lo, 32 * nb + 4 * G + c, O, inv[32 * nb + 4 * G + c]);
-                }
-                continue;
-            }
+        for (int nb = wave; nb < N / 32; nb += waves) {
+            floatx16 acc[MI][1];
+            multiply<MI, 1, kSums>(a.planes[2] + (long)nb * (O >> 5) * 1024, w_lo, O, xh, 32 * O, x_lo, lane, acc);
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const float4 iw = *reinterpret_cast<const float4*>(inv + 32 * nb + 8 * t + 4 * G);
-                *reinterpret_cast<float4*>(out + 8 * t) =
-                    make_float4(acc[0][4 * t] * row_isx * iw.x, acc[0][4 * t + 1] * row_isx * iw.y,
-                                acc[0][4 * t + 2] * row_isx * iw.z, acc[0][4 * t + 3] * row_isx * iw.w);
+            for (int mi = 0; mi < MI; mi++) {
+                if (!live(mi)) continue;
+                float* out = a.y + row_of(mi, m) * N + 32 * nb + 4 * G;
+                if (odd[mi]) {
+#pragma unroll 1
+                    for (int q = 0; q < 16; q++) {
+                        const int c = 8 * (q / 4) + q % 4, n = 32 * nb + 4 * G + c;
+                        out[c] = lds_row_in_fp32(xh + mi * 32 * O, x_lo, m, a.planes[2], w_lo, n, O, inv[n]);
+                    }
+                    continue;
+                }
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    const float4 iw = *reinterpret_cast<const float4*>(inv + 32 * nb + 8 * t + 4 * G);
+                    *reinterpret_cast<float4*>(out + 8 * t) =
+                        make_float4(acc[mi][0][4 * t] * isx[mi] * iw.x, acc[mi][0][4 * t + 1] * isx[mi] * iw.y,
+                                    acc[mi][0][4 * t + 2] * isx[mi] * iw.z, acc[mi][0][4 * t + 3] * isx[mi] * iw.w);
+                }
             }
         }
     }
 }
 
-template <int MI, int MODE, bool DUAL>
+template <int MI, int NI, int MODE, bool DUAL>
 int launch(const MlpArgs& a, hipStream_t st) {
-    const auto kernel = mlp_f16x2_kernel<MI, MODE, DUAL>;
+    const auto kernel = mlp_f16x2_kernel<MI, NI, MODE, DUAL>;
     const int widest = a.K > a.O ? a.K : a.O;
-    const size_t lds = (size_t)32 * MI * widest * 4 + (kMaxWaves * 32 * MI + kMaxDim) * sizeof(float);
+    const size_t lds = (size_t)32 * MI * widest * 4 + (kMaxWaves / NI * 32 * MI + kMaxDim) * sizeof(float);
     // more than 64 KB of dynamic LDS has to be asked for (per device, so on every call)
     if (lds > 65536) MG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    const long tiles = ceil_div(a.R, DUAL ? 32 : 32 * MI);
+    const long tiles = ceil_div(a.R, DUAL ? 16 : 32 * MI);
     MG_REQUIRE(tiles <= 0x7fffffffL, "mg_mlp_f16x2: grid too large (rows=%ld)", a.R);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(2 * a.O), lds, st, a);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(2 * a.O / NI), lds, st, a);
     return check_launch("mg_mlp_f16x2");
 }
 
 template <int MODE>
 int choose(const MlpArgs& a, bool dual, hipStream_t st) {
-    if constexpr (MODE != kInfer)
-        if (dual) return launch<2, MODE, true>(a, st);
-    // 32 rows a workgroup while the chip holds all of them at once, 64 beyond (the weights are read half as often):
-    // 128 -> 512 on 8192 rows 42 against 53 us, on 16 336 83 against 69; 128 -> 128 on 16 336 14.5 against 18.0
-    const int mi = ceil_div(a.R, 32) * (a.O / 32) > 256 * kMaxWaves ? 2 : 1;
-    return mi == 2 ? launch<2, MODE, false>(a, st) : launch<1, MODE, false>(a, st);
+    if constexpr (MODE == kInfer) {
+        // 32 rows a workgroup while the chip holds all of them at once, 64 beyond (the weights are read half as often):
+        // 128 -> 512 on 8192 rows 42 against 53 us, on 16 336 83 against 69; 128 -> 128 on 16 336 14.5 against 18.0
+        if (ceil_div(a.R, 32) * (a.O / 32) > 256 * kMaxWaves) return launch<2, 1, MODE, false>(a, st);
+        return launch<1, 1, MODE, false>(a, st);
+    } else {
+        // The passes over memory between the layers are longer here (z and h, or z and the gradients): from more tiles than CUs on two
+        // workgroups of half as many waves share a CU, and one multiplies while the other writes.  128 -> 512, forward / adjoint, one
+        // / two workgroups: 8192 rows 58 / 54 and 62 / 56 us, 12 000 96 / 96 and 94 / 88, 16 384 119 / 108 and 102 / 95,
+        // 2 x 39 000 with tangents 576 / 554 and 528 / 501.
+        const long tiles = ceil_div(a.R, dual ? 16 : 32);
+        if (a.O > 256 && a.O % 64 == 0 && tiles > 256) return dual ? launch<1, 2, MODE, true>(a, st) : launch<1, 2, MODE, false>(a, st);
+        return dual ? launch<1, 1, MODE, true>(a, st) : launch<1, 1, MODE, false>(a, st);
+    }
 }
 
 int fill(MlpArgs& a, const void* const* packed, int K, int O, int N) {
@@ -480,6 +534,7 @@ int mg_mlp_f16x2_adjoint(const mg_mlp_f16x2_grad* p, mg_stream_t stream) {
     a.K = a.O = p->dim;
     a.N = p->dim_in;
     a.y = p->dx;
+    a.x_max = p->dy_rowmax;
     for (int l = 0; l < 2; l++) {                                  // met in reverse
         a.z_in[l] = p->z[1 - l];
         a.h[l] = p->dz[1 - l];

@@ -4,6 +4,7 @@
 // node-sized launches was bound by.  No arithmetic happens here.
 #include "torch_common.hpp"
 
+#include <algorithm>
 #include <atomic>
 #include <climits>
 #include <limits>
@@ -488,6 +489,8 @@ using Tensors = std::vector<at::Tensor>;
 
 const std::vector<int> kSiluMlp{kActSilu, kActSilu, kActNone};
 
+bool aligned_all(const Tensors& t) { return std::all_of(t.begin(), t.end(), [](const at::Tensor& v) { return aligned16(v); }); }
+
 // Whether the three layers of an MLP on x (rows, k) go through one kernel (k: W[0]'s columns after zero padding).
 // A workgroup reads all three weights whatever the number of rows, about 30 us of a kernel at 128 -> 512 -> 512 -> 512 and 10 us
 // at 128 -> 128: for wide layers of few rows the three launches that split the reduction of each over the chip are faster (us,
@@ -496,12 +499,12 @@ const std::vector<int> kSiluMlp{kActSilu, kActSilu, kActNone};
 // at 16 384; 128 -> 128 9.9 / 14.2 at 64).  Distance from float64 at 128 -> 512: 2.3e-7 against 2.2..2.5e-7 with split
 // reductions, 2.75e-7 against 4.1e-7 at 16 336 rows.
 constexpr int64_t kMlpWide = 256, kMlpWideRows = 1024;
-bool mlp_takes(int64_t rows, int64_t k, const Tensors& W, const Tensors& b, const at::Tensor& x) {
+bool mlp_takes(int64_t rows, int64_t k, const Tensors& W, const at::Tensor& x) {
     const int64_t dim = W[0].size(0);
     if (mg_get_linear_mode() != kModeF16x2 || rows < (dim > kMlpWide ? kMlpWideRows : 1) || k < 64 || dim < 64 || !mg_mlp_f16x2_supported((int)k, (int)dim))
         return false;
     for (size_t l = 0; l < 3; l++)
-        if (W[l].size(0) != dim || (l > 0 && W[l].size(1) != dim) || !aligned16(b[l])) return false;
+        if (W[l].size(0) != dim || (l > 0 && W[l].size(1) != dim)) return false;
     return aligned16(x);
 }
 
@@ -526,7 +529,7 @@ at::Tensor mlp_fused(const at::Tensor& x, const Tensors& W, const Tensors& b) {
 // a chain of linears with fused bias and activation; the row bounds the split-fp16 layers scale by travel as
 // mul * base + add through the layers' norms, so that only the first layer ever looks at the data for them
 at::Tensor chain(at::Tensor h, const Tensors& W, const Tensors& b, const std::vector<int>& act, Bound bound) {
-    if (act == kSiluMlp && mlp_takes(h.size(0), h.size(1), W, b, h)) return mlp_fused(h, W, b);
+    if (act == kSiluMlp && mlp_takes(h.size(0), h.size(1), W, h) && aligned_all(b)) return mlp_fused(h, W, b);
     for (size_t k = 0; k < W.size(); k++) {
         const int64_t rows = h.size(0), dim_in = W[k].size(1), dim_out = W[k].size(0);
         at::Tensor y = floats(h, {rows, dim_out});
@@ -637,7 +640,7 @@ at::Tensor filter_grid(const at::Tensor& enc, const at::Tensor& unit, const Tens
     TORCH_CHECK(k > W[0].size(1) && k % 32 == 0 && mg_get_linear_mode() == kModeF16x2 && aligned16(enc),
                 "filter_grid: encodings of a wrong width");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(enc.device());
-    if (mlp_takes(rows, k, W, b, enc)) return mlp_fused(enc, W, b);
+    if (mlp_takes(rows, k, W, enc) && aligned_all(b)) return mlp_fused(enc, W, b);
     at::Tensor h = floats(enc, {rows, W[0].size(0)});
     const OptTensor b0(b[0]);
     run_f16x2(W[0], k, fp(enc), rows, Bound{OptTensor(unit)}, b0, kActSilu, false, 1, h, nullptr, false);
@@ -828,12 +831,49 @@ std::pair<at::Tensor, OptTensor> rows_wgrad(const at::Tensor& dy, const at::Tens
     return {dW, want_bias ? OptTensor(dy.narrow(0, 0, bias_rows).sum(0)) : OptTensor()};
 }
 
+// Wide layers on values and tangents together: the one kernel has one accumulator for the large products there, 2.75e-7 from
+// float64 where the split reductions of few rows are at 2.5e-7: it takes over where those end (4.1e-7 beyond).
+bool mlp_dual_takes(int64_t rows, const Tensors& W, bool dual) {
+    const int dim = (int)W[0].size(0);
+    return !dual || dim <= kMlpWide || !mg_tensor_linear_f16x2_splits_k(rows, dim, dim);
+}
+
 // Linear, SiLU, Linear, SiLU, Linear on S = [x; x_t] (R or 2 R rows): y and what the adjoint reads again
 std::pair<at::Tensor, std::vector<OptTensor>> mlp_rows_fwd(const at::Tensor& S, int64_t R, OptTensor bound, const Tensors& W,
                                                            const Tensors& b, bool train) {
     check_chain(S, W, b, kSiluMlp);
     const bool dual = S.size(0) != R;
     if (train) pack_ahead({W[0], W[1], W[2], W[0].t(), W[1].t(), W[2].t()});
+    if (mlp_takes(S.size(0), S.size(1), W, S) && aligned_all(b) && mlp_dual_takes(S.size(0), W, dual)) {
+        const int64_t rows = S.size(0), dim = W[0].size(0);
+        mg_mlp_f16x2 a{};
+        at::Tensor y = floats(S, {rows, dim});
+        if (!bound.has_value()) {
+            bound = floats(S, {rows, 1});
+            a.x_rowmax = fp(*bound);
+        }
+        std::vector<OptTensor> saved{bound};
+        Tensors planes;
+        for (int l = 0; l < 3; l++) {
+            planes.push_back(packed_f16x2(W[l], W[l].size(1)));
+            a.packed_W[l] = planes[l].data_ptr();
+            a.bias[l] = fp(b[l]);
+            if (l == 2) break;
+            at::Tensor z = floats(S, {rows, dim}), m = floats(S, {rows, 1}), h = floats(S, {rows, dim});
+            a.z[l] = fp(z);
+            a.h[l] = fp(h);
+            a.h_rowmax[l] = fp(m);
+            saved.insert(saved.end(), {OptTensor(z), OptTensor(m), OptTensor(h)});
+        }
+        a.x = fp(S);
+        a.rows = R;
+        a.dual = dual;
+        a.dim_in = (int)S.size(1);
+        a.dim = (int)dim;
+        a.y = fp(y);
+        check(mg_mlp_f16x2_forward(&a, stream_of(S)));
+        return {y, saved};
+    }
     if (!bound.has_value() && S.size(1) >= 64) bound = row_absmax(S);
     std::vector<OptTensor> saved{bound};
     at::Tensor h = S;
@@ -854,15 +894,50 @@ std::tuple<OptTensor, Tensors> mlp_rows_bwd(at::Tensor g, OptTensor g_bound, con
     const bool dual = S.size(0) != R;
     Tensors params(6);
     OptTensor g_x;
+    auto weight_grads = [&](int l, const at::Tensor& dz, const OptTensor& dz_bound) {
+        if (!want_params) return;
+        auto [dW, db] = rows_wgrad(dz, l == 0 ? S : *saved[3 * l], R, true, dz_bound, l == 0 ? saved[0] : saved[3 * l - 1]);
+        params[2 * l] = dW;
+        params[2 * l + 1] = *db;
+    };
+    const int64_t dim = W[0].size(0);
+    if (saved[0].has_value() && g.size(1) == dim && aligned16(g) && mlp_takes(S.size(0), S.size(1), W, S) &&
+        mlp_dual_takes(S.size(0), W, dual)) {
+        const int64_t rows = S.size(0);
+        mg_mlp_f16x2_grad a{};
+        if (!g_bound.has_value()) {
+            g_bound = floats(g, {rows, 1});
+            a.dy_rowmax = fp(*g_bound);
+        }
+        at::Tensor dz[2], m[2];
+        Tensors planes;
+        for (int l = 0; l < 3; l++) {
+            planes.push_back(packed_f16x2(W[l].t(), W[l].size(0)));
+            a.packed_Wt[l] = planes[l].data_ptr();
+            if (l == 2) break;
+            dz[l] = floats(g, {rows, dim});
+            m[l] = floats(g, {rows, 1});
+            a.z[l] = fp(*saved[3 * l + 1]);
+            a.dz[l] = fp(dz[l]);
+            a.dz_rowmax[l] = fp(m[l]);
+        }
+        if (want_x) {
+            g_x = floats(S, S.sizes());
+            a.dx = fp(*g_x);
+        }
+        a.dy = fp(g);
+        a.rows = R;
+        a.dual = dual;
+        a.dim_in = (int)S.size(1);
+        a.dim = (int)dim;
+        check(mg_mlp_f16x2_adjoint(&a, stream_of(g)));
+        weight_grads(2, g, g_bound);
+        for (int l = 1; l >= 0; l--) weight_grads(l, dz[l], OptTensor(m[l]));
+        return {g_x, params};
+    }
     for (int l = 2; l >= 0; l--) {
         if (!g_bound.has_value()) g_bound = row_absmax(g);
-        const at::Tensor& in = l == 0 ? S : *saved[3 * l];
-        const OptTensor& in_bound = l == 0 ? saved[0] : saved[3 * l - 1];
-        if (want_params) {
-            auto [dW, db] = rows_wgrad(g, in, R, true, g_bound, in_bound);
-            params[2 * l] = dW;
-            params[2 * l + 1] = *db;
-        }
+        weight_grads(l, g, g_bound);
         if (l == 0) {
             if (want_x) g_x = rows_linear(W[0].t(), OptTensor(), g, 0, Bound{g_bound});
             break;

@@ -22,10 +22,13 @@ def _formula(x, W, b):
     return h
 
 
-def _assert_rows(y, ref, what):
+def _assert_rows(y, ref, what, f32=None):
     """2-norm of a row's difference against the row's: three layers, each rounding its operands to 22 bits and its sums and
-    activation to 24, err by 5e-7 at most; measured 2e-7 .. 3e-7 over all rows."""
-    err = (y.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    activation to 24, err by 5e-7 at most; measured 2e-7 .. 3e-7 over all rows.  f32: the formula in float32, where a row's terms may
+    cancel (the adjoint's g f' + g_t z_t f''): twice its distance is what the row's conditioning adds."""
+    def error(t):
+        return (t.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    err = error(y) - (0 if f32 is None else 2 * error(f32))
     assert float(err.max()) <= 1.5e-6, (what, float(err.max()))
 
 
@@ -66,3 +69,62 @@ def test_mlp_rows_and_weights_beyond_the_pieces(ops, rows, dim_in, dim):
     W[2][5, 3] = 0.5
     W[0][7, 2] = NAN
     assert bool(torch.isnan(ops.linear_chain(x, W, b, ACTS, None)).all())
+
+
+def _dual_formula(x, x_t, W, b):
+    """y and its tangent in float64, differentiable."""
+    h, h_t = x, x_t
+    for k in range(3):
+        z, z_t = h @ W[k].t() + b[k], None if h_t is None else h_t @ W[k].t()
+        if k < 2:
+            s = torch.sigmoid(z)
+            h, h_t = z * s, None if z_t is None else (s + z * s * (1 - s)) * z_t
+        else:
+            h, h_t = z, z_t
+    return h, h_t
+
+
+# (rows at the edges of the tiles of 32 rows, 16 with tangents, and on both sides of one workgroup per CU)
+@pytest.mark.parametrize("rows, dim_in, dim, dual", [(1, 64, 64, False), (33, 128, 256, False), (1025, 96, 512, False), (8300, 64, 320, False),
+                                                     (1, 64, 96, True), (17, 512, 128, True), (1000, 256, 192, True), (2300, 128, 512, True),
+                                                     (4200, 64, 384, True), (4100, 64, 288, True)])
+def test_mlp_adjoint_in_one_kernel(ops, rows, dim_in, dim, dual):
+    W, b = _weights(dim_in, dim)
+    g = torch.Generator().manual_seed(rows)
+    S = (torch.randn(2 * rows, dim_in, generator=g) * torch.exp(torch.randn(2 * rows, 1, generator=g))).cuda()
+    G = torch.randn(2 * rows, dim, generator=g).cuda()
+    x, x_t, gy, gy_t = S[:rows], S[rows:] if dual else None, G[:rows], G[rows:] if dual else None
+    y, y_t, saved = ops.mlp_silu_fwd(x, x_t, None, W, b, True)
+    g_x, g_xt, params = ops.mlp_silu_bwd(gy, gy_t, x, x_t, W, saved, True, True)
+
+    def formula(dt):
+        leaves = [t.detach().clone().to(dt).requires_grad_() for t in (x, *W, *b)] + ([x_t.clone().to(dt).requires_grad_()] if dual else [])
+        ref, ref_t = _dual_formula(leaves[0], leaves[7] if dual else None, leaves[1:4], leaves[4:7])
+        loss = (ref * gy.to(dt)).sum() + ((ref_t * gy_t.to(dt)).sum() if dual else 0)
+        grads = torch.autograd.grad(loss, leaves)
+        return [ref.detach(), grads[0]] + ([ref_t.detach(), grads[7]] if dual else []), grads
+
+    (ref, grads), (ref32, _) = formula(torch.float64), formula(torch.float32)
+    for what, a, r, r32 in zip(("y", "g_x", "y_t", "g_xt"), (y, g_x, y_t, g_xt), ref, ref32):
+        _assert_rows(a, r, (what, rows, dim_in, dim, dual), r32)
+    for k in range(3):                                           # (sums over rows: the whole matrix against its norm)
+        for a, r in ((params[2 * k], grads[1 + k]), (params[2 * k + 1], grads[4 + k])):
+            assert float((a.double() - r).norm() / r.norm()) <= 4e-6, (k, rows, dim_in, dim, dual)
+    no_x, _, _ = ops.mlp_silu_bwd(gy, gy_t, x, x_t, W, saved, False, True)
+    assert no_x is None
+
+
+@pytest.mark.parametrize("rows, dim", [(50, 64), (1100, 512), (8300, 512)])
+def test_mlp_adjoint_of_a_row_beyond_the_pieces(ops, rows, dim):
+    W, b = _weights(64, dim)
+    g = torch.Generator().manual_seed(2)
+    x, gy = torch.randn(rows, 64, generator=g).cuda(), torch.randn(rows, dim, generator=g).cuda()
+    y, _, saved = ops.mlp_silu_fwd(x, None, None, W, b, True)
+    clean, _, _ = ops.mlp_silu_bwd(gy, None, x, None, W, saved, True, False)
+    gy[rows - 2, 3], gy[5] = INF, gy[5] * 2.0 ** 100
+    g_x, _, _ = ops.mlp_silu_bwd(gy, None, x, None, W, saved, True, False)
+    same = torch.ones(rows, dtype=torch.bool, device="cuda")
+    same[[5, rows - 2]] = False
+    assert torch.equal(g_x[same], clean[same])
+    assert not bool(torch.isfinite(g_x[rows - 2]).any())
+    assert float((g_x[5].double() * 2.0 ** -100 - clean[5].double()).norm() / clean[5].double().norm()) <= 1.5e-6
