@@ -329,13 +329,13 @@ __global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const
                         for (int i = 0; i < 4; i++) {
                             if constexpr (DUAL) {                  // this lane: value and tangent of one of the two columns
                                 swap_rows(v[0][i], v[1][i]);
-                                const Silu s = silu(v[0][i]);
+                                const Silu s = silu_short(v[0][i]);
                                 v[0][i] = s.f;
                                 v[1][i] *= s.d1;
                                 swap_rows(v[0][i], v[1][i]);
                             } else {
-                                v[0][i] = silu(v[0][i]).f;
-                                v[1][i] = silu(v[1][i]).f;
+                                v[0][i] = silu_short(v[0][i]).f;
+                                v[1][i] = silu_short(v[1][i]).f;
                             }
                         }
                         put(a.h[l]);
@@ -351,13 +351,13 @@ __global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const
                             if constexpr (DUAL) {
                                 swap_rows(v[0][i], v[1][i]);
                                 swap_rows(z[0][i], z[1][i]);
-                                const Silu s = silu(z[0][i]);
+                                const Silu s = silu_short(z[0][i]);
                                 v[0][i] = v[0][i] * s.d1 + v[1][i] * z[1][i] * s.d2;
                                 v[1][i] *= s.d1;
                                 swap_rows(v[0][i], v[1][i]);
                             } else {
-                                v[0][i] *= silu(z[0][i]).d1;
-                                v[1][i] *= silu(z[1][i]).d1;
+                                v[0][i] *= silu_short(z[0][i]).d1;
+                                v[1][i] *= silu_short(z[1][i]).d1;
                             }
                         }
                         put(a.h[l]);
