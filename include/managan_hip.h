@@ -635,14 +635,22 @@ int mg_painn_grid_node_grad(const int* row_ptr, const int* order, const int* src
                             mg_stream_t stream);
 /* row[e]: the grid row below an edge's length */
 int mg_painn_grid_rows(const float* r_ij, long n_edges, int table_rows, float period, int* row, mg_stream_t stream);
-/* d_table (table_rows, 4n).  order / bucket_ptr: the edges sorted by mg_painn_grid_rows; actv_sliced as in
- * mg_painn_table_message_sliced. */
+/* The same with the edges of a graph (row_ptr over n_nodes sources) taken source by source in node_order: row and edge per position.
+ * Edges behind the last row follow as they come. */
+int mg_painn_grid_rows_by_node_workspace_bytes(int n_nodes, size_t* bytes /* host */);
+int mg_painn_grid_rows_by_node(const float* r_ij, long n_edges, const int* row_ptr, const int* node_order, int n_nodes, int table_rows,
+                               float period, void* workspace, int* row, int* edge, mg_stream_t stream);
+/* d_table (table_rows, 4n).  order / bucket_ptr: the edges sorted by mg_painn_grid_rows (by_node: near each other in space near each
+ * other in their row's bucket, which the gathers of node rows gain from); actv_sliced as in mg_painn_table_message_sliced. */
 int mg_painn_grid_table_grad(const int* order, const int* bucket_ptr, const int* src, const int* dst, int n_nodes, long n_edges,
                              const float* r_ij, int table_rows, float period, float epsilon, const float* g_v, const float* g_a,
                              const float* actv_sliced, const float* v, int n, void* workspace, float* d_table, mg_stream_t stream);
 /* order: the positions of keys (0 .. key_limit - 1) in the order of a stable sort; sorted_keys: the keys in that order. */
 int mg_sort_by_key_workspace_bytes(long count, size_t* bytes /* host */);
 int mg_sort_by_key(const int* keys, long count, int key_limit, void* workspace, int* order, int* sorted_keys, mg_stream_t stream);
+/* the same with `order` the values that go with the keys (NULL: their positions) */
+int mg_sort_values_by_key(const int* keys, const int* values, long count, int key_limit, void* workspace, int* order, int* sorted_keys,
+                          mg_stream_t stream);
 
 /* The PaiNN layers under differentiation (archs/meanflow_painn8.py:25-100; the meanflow loss, :274-296): the passes between the
  * linear maps, forward and adjoint.  dual != 0: every array holds `rows` rows of values and then `rows` rows of forward-mode

@@ -71,6 +71,62 @@ __global__ void __launch_bounds__(256) grid_row_kernel(const float* __restrict__
     if (e < E) row[e] = (int)floorf(place(r_ij[3 * e], r_ij[3 * e + 1], r_ij[3 * e + 2], inv_h, eps).u) & mask;
 }
 
+// The same with the edges taken in the order of their sources in node_order (cells of the neighbour search): row and edge per
+// position.  Neighbours in space then stay neighbours inside a grid row's bucket, and so do the node rows its kernel gathers.
+// first[slot]: position of a slot's first edge inside its block of 256 slots, block_edges: the block's edges.
+constexpr int kSlotBlock = 256, kTailBlocks = 64;
+__global__ void __launch_bounds__(kSlotBlock) slot_starts_kernel(const int* __restrict__ row_ptr, const int* __restrict__ node_order,
+                                                                 long n_nodes, int* __restrict__ first, int* __restrict__ block_edges) {
+    __shared__ int wave_sum[kSlotBlock / kWave];
+    const long slot = (long)blockIdx.x * kSlotBlock + threadIdx.x;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    int own = 0;
+    if (slot < n_nodes) {
+        const long node = min(max((long)node_order[slot], 0L), n_nodes - 1);
+        own = max(row_ptr[node + 1] - row_ptr[node], 0);
+    }
+    int sum = own;
+    for (int d = 1; d < kWave; d <<= 1) {
+        const int up = __shfl_up(sum, d);
+        if (lane >= d) sum += up;
+    }
+    if (lane == kWave - 1) wave_sum[wave] = sum;
+    __syncthreads();
+    int before = 0, total = 0;
+    for (int w = 0; w < kSlotBlock / kWave; w++) {
+        if (w < wave) before += wave_sum[w];
+        total += wave_sum[w];
+    }
+    if (slot < n_nodes) first[slot] = before + sum - own;
+    if (threadIdx.x == 0) block_edges[blockIdx.x] = total;
+}
+// a wave per slot; the last kTailBlocks blocks take edges behind the last row, as they come
+__global__ void __launch_bounds__(256) grid_row_by_node_kernel(const float* __restrict__ r_ij, const int* __restrict__ row_ptr,
+                                                               const int* __restrict__ node_order, long n_nodes, long E,
+                                                               const int* __restrict__ first, const int* __restrict__ block_edges,
+                                                               int mask, float inv_h, float eps, int* __restrict__ row,
+                                                               int* __restrict__ edge) {
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    auto put = [&](long p, long e) {
+        row[p] = (int)floorf(place(r_ij[3 * e], r_ij[3 * e + 1], r_ij[3 * e + 2], inv_h, eps).u) & mask;
+        edge[p] = (int)e;
+    };
+    const long slot_blocks = gridDim.x - kTailBlocks;
+    if (blockIdx.x >= slot_blocks) {
+        for (long p = max(row_ptr[n_nodes], 0) + (blockIdx.x - slot_blocks) * 256 + threadIdx.x; p < E; p += 256 * kTailBlocks) put(p, p);
+        return;
+    }
+    const long slot = (long)blockIdx.x * 4 + wave;
+    if (slot >= n_nodes) return;
+    int base = 0;
+    for (int b = lane; b < slot / kSlotBlock; b += kWave) base += block_edges[b];
+    for (int d = 1; d < kWave; d <<= 1) base += __shfl_xor(base, d);
+    const long node = min(max((long)node_order[slot], 0L), n_nodes - 1);
+    const long lo = max(row_ptr[node], 0), hi = min((long)row_ptr[node + 1], E), at = (long)base + first[slot];
+    for (long e = lo + lane; e < hi; e += kWave)
+        if (at + e - lo < E) put(at + e - lo, e);
+}
+
 // ------------------------------------------------------------------------------------------------ gradients of actv and v
 // The mapping of painn_table_message_lds_kernel: a workgroup holds one slice of 16 channels of the grid in LDS, a wave takes 16
 // edges of its node per step, 4 lanes x 4 channels each.  Bound by vector issue, like that kernel.
@@ -163,7 +219,10 @@ __global__ void __launch_bounds__(1024) grid_node_grad_kernel(
 // part[((row splits + s) 4 + j) 4n + k n + c]: piece s of the edges of a grid row, in order; a wave takes 16 edges per step as
 // above, its 64 sums per lane are added over the slots at the end and over the 4 waves in wave order.  Slices are the fastest
 // block index (one slice per XCD at n = 128), pieces the slowest: the blocks that run together read the rows of the same part
-// of the nodes.  Bound by those reads (11 x 16 bytes per lane and edge against 64 multiply-adds).
+// of the nodes.  Bound by those reads (11 x 16 bytes per lane and edge against 64 multiply-adds): 9.0 GB in 480 us at 1.6 M edges, n = 128,
+// of the 20 TB/s that gathers of this size and alignment reach from the L2 (16 384 x 256 bytes: 21).  With the edges of a bucket in
+// the order of their atoms' numbers, whose neighbours are anywhere, 621 us.  32-bit offsets and a peeled last step (four waves per
+// SIMD for three) made it slower, 600 us.
 __global__ void __launch_bounds__(256) grid_row_grad_kernel(const int* __restrict__ bucket_ptr, const float4* __restrict__ rec,
                                                             long E, int rows, int splits, long n_nodes,
                                                             const float* __restrict__ actv_s, const float* __restrict__ v,
@@ -357,8 +416,10 @@ __global__ void __launch_bounds__(256) sort_scatter_kernel(const int* __restrict
 }
 
 int splits_of(int rows, long E) {
-    // pieces of about 768 edges: 12 steps of the 4 waves, against which adding 64 sums over the slots is a fifth
-    long s = ceil_div(E, 768L * rows);
+    // pieces of about 400 edges: 6 steps of the 4 waves, against which adding 64 sums over the slots is a third; the fewer edges, the
+    // smaller the part of space whose node rows the pieces that run together read (1.6 M edges, pieces of 200 / 400 / 768 / 1600: 526,
+    // 479, 504, 716 us, their sums 22, 11, 7, 5)
+    long s = ceil_div(E, 400L * rows);
     return (int)(s < 1 ? 1 : (s > 16 ? 16 : s));
 }
 
@@ -420,6 +481,30 @@ int mg_painn_grid_rows(const float* r_ij, long n_edges, int table_rows, float pe
     return check_launch("mg_painn_grid_rows");
 }
 
+int mg_painn_grid_rows_by_node_workspace_bytes(int n_nodes, size_t* bytes) {
+    MG_REQUIRE(bytes && n_nodes >= 0, "mg_painn_grid_rows_by_node_workspace_bytes: bad argument");
+    *bytes = ((size_t)n_nodes + ceil_div(n_nodes, kSlotBlock)) * sizeof(int);
+    return MG_OK;
+}
+
+int mg_painn_grid_rows_by_node(const float* r_ij, long n_edges, const int* row_ptr, const int* node_order, int n_nodes, int table_rows,
+                               float period, void* workspace, int* row, int* edge, mg_stream_t stream) {
+    MG_REQUIRE(n_edges >= 0 && n_edges < (1L << 31) && n_nodes >= 0 && (n_nodes > 0 || n_edges == 0) && period > 0.f && table_rows >= 4 &&
+                   (table_rows & (table_rows - 1)) == 0,
+               "mg_painn_grid_rows_by_node: bad argument");
+    if (n_edges == 0) return MG_OK;
+    MG_REQUIRE(r_ij && row_ptr && node_order && workspace && row && edge, "mg_painn_grid_rows_by_node: null pointer");
+    int* first = static_cast<int*>(workspace);
+    int* block_edges = first + n_nodes;
+    hipStream_t st = (hipStream_t)stream;
+    hipLaunchKernelGGL(slot_starts_kernel, dim3((unsigned)ceil_div(n_nodes, kSlotBlock)), dim3(kSlotBlock), 0, st, row_ptr, node_order,
+                       (long)n_nodes, first, block_edges);
+    hipLaunchKernelGGL(grid_row_by_node_kernel, dim3((unsigned)(ceil_div(n_nodes, 4) + kTailBlocks)), dim3(256), 0, st, r_ij, row_ptr,
+                       node_order, (long)n_nodes, n_edges, (const int*)first, (const int*)block_edges, table_rows - 1,
+                       (float)table_rows / period, 1.0f, row, edge);
+    return check_launch("mg_painn_grid_rows_by_node");
+}
+
 int mg_painn_grid_table_grad(const int* order, const int* bucket_ptr, const int* src, const int* dst, int n_nodes, long n_edges,
                              const float* r_ij, int table_rows, float period, float epsilon, const float* g_v, const float* g_a,
                              const float* actv_sliced, const float* v, int n, void* workspace, float* d_table, mg_stream_t stream) {
@@ -450,6 +535,11 @@ int mg_sort_by_key_workspace_bytes(long count, size_t* bytes) {
 }
 
 int mg_sort_by_key(const int* keys, long count, int key_limit, void* workspace, int* order, int* sorted_keys, mg_stream_t stream) {
+    return mg_sort_values_by_key(keys, nullptr, count, key_limit, workspace, order, sorted_keys, stream);
+}
+
+int mg_sort_values_by_key(const int* keys, const int* values, long count, int key_limit, void* workspace, int* order, int* sorted_keys,
+                          mg_stream_t stream) {
     MG_REQUIRE(count >= 0 && count < (1L << 31) && key_limit >= 1, "mg_sort_by_key: bad argument");
     if (count == 0) return MG_OK;
     MG_REQUIRE(keys && workspace && order && sorted_keys, "mg_sort_by_key: null pointer");
@@ -460,7 +550,7 @@ int mg_sort_by_key(const int* keys, long count, int key_limit, void* workspace, 
     int *spare_keys = totals + kDigits, *spare_values = spare_keys + count;
     int passes = 1;
     while (passes < 4 && ((long)key_limit - 1) >> (kDigitBits * passes)) passes++;
-    const int *k_in = keys, *v_in = nullptr;
+    const int *k_in = keys, *v_in = values;
     for (int p = 0; p < passes; p++) {
         // the last pass ends in the caller's arrays
         const bool to_out = (passes - 1 - p) % 2 == 0;

@@ -1175,17 +1175,20 @@ std::tuple<std::vector<OptTensor>, Tensors> painn_update_train_bwd(const at::Ten
     return {g_x, params};
 }
 
-// (order, sorted keys) of a stable sort of int32 keys in 0 .. limit - 1
-std::pair<at::Tensor, at::Tensor> sort_by_key(const at::Tensor& keys, int64_t limit) {
-    check_input(keys, "keys", at::kInt);
-    c10::hip::HIPGuardMasqueradingAsCUDA guard(keys.device());
+// (order, sorted keys) of a stable sort of int32 keys in 0 .. limit - 1; values: what order holds in the place of positions
+std::pair<at::Tensor, at::Tensor> sort_values_by_key(const at::Tensor& keys, const OptTensor& values, int64_t limit) {
     at::Tensor order = at::empty_like(keys), sorted = at::empty_like(keys);
     size_t n = 0;
     check(mg_sort_by_key_workspace_bytes(keys.numel(), &n));
     at::Tensor ws = bytes_like(keys, n);
-    check(mg_sort_by_key(keys.data_ptr<int>(), keys.numel(), (int)limit, ws.data_ptr(), order.data_ptr<int>(), sorted.data_ptr<int>(),
-                         stream_of(keys)));
+    check(mg_sort_values_by_key(keys.data_ptr<int>(), values.has_value() ? values->data_ptr<int>() : nullptr, keys.numel(), (int)limit,
+                                ws.data_ptr(), order.data_ptr<int>(), sorted.data_ptr<int>(), stream_of(keys)));
     return {order, sorted};
+}
+std::pair<at::Tensor, at::Tensor> sort_by_key(const at::Tensor& keys, int64_t limit) {
+    check_input(keys, "keys", at::kInt);
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(keys.device());
+    return sort_values_by_key(keys, OptTensor(), limit);
 }
 
 // (d_table, d_actv, d_v) of the message interpolated from its grid; each only if wanted
@@ -1195,16 +1198,17 @@ std::tuple<OptTensor, OptTensor, OptTensor> painn_grid_message_bwd(const at::Ten
                                                                    const at::Tensor& src, const at::Tensor& dst,
                                                                    const at::Tensor& row_ptr, const OptTensor& order,
                                                                    const OptTensor& node_order, double period, double epsilon,
-                                                                   bool want_table, bool want_actv, bool want_v) {
+                                                                   bool want_table, bool want_actv, bool want_v,
+                                                                   const OptTensor& src_row_ptr) {
     for (const at::Tensor& t : {table, actv, actv_sliced, v, r_ij, g_v, g_a}) check_input(t, "operand of the message");
     for (const at::Tensor& t : {src, dst, row_ptr}) check_input(t, "index", at::kInt);
-    for (const OptTensor& t : {order, node_order})
+    for (const OptTensor& t : {order, node_order, src_row_ptr})
         if (t.has_value()) check_input(*t, "order", at::kInt);
     const int64_t N = v.size(0), n = v.size(1), E = r_ij.size(0), rows = table.size(0);
     TORCH_CHECK(actv.numel() == N * 4 * n && actv_sliced.numel() == N * 4 * n && v.numel() == N * n * 3 && table.size(1) == 4 * n &&
                     g_v.numel() == N * n * 3 && g_a.numel() == N * n && r_ij.numel() == 3 * E && src.numel() == E && dst.numel() == E &&
                     row_ptr.numel() == N + 1 && (!order.has_value() || order->numel() == E) &&
-                    (!node_order.has_value() || node_order->numel() == N),
+                    (!node_order.has_value() || node_order->numel() == N) && (!src_row_ptr.has_value() || src_row_ptr->numel() == N + 1),
                 "painn_grid_message_bwd: operand sizes");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(v.device());
     const mg_stream_t st = stream_of(v);
@@ -1223,8 +1227,18 @@ std::tuple<OptTensor, OptTensor, OptTensor> painn_grid_message_bwd(const at::Ten
     if (want_table) {
         d_table = floats(v, table.sizes());
         at::Tensor key = at::empty({E}, src.options()), ptr = at::empty({rows + 1}, src.options());
-        check(mg_painn_grid_rows(fp(r_ij), E, (int)rows, (float)period, key.data_ptr<int>(), st));
-        auto [by_row, sorted] = sort_by_key(key, rows);
+        OptTensor edge;
+        if (node_order.has_value() && src_row_ptr.has_value()) {
+            edge = at::empty({E}, src.options());
+            size_t bytes = 0;
+            check(mg_painn_grid_rows_by_node_workspace_bytes((int)N, &bytes));
+            at::Tensor starts = bytes_like(v, bytes);
+            check(mg_painn_grid_rows_by_node(fp(r_ij), E, src_row_ptr->data_ptr<int>(), node_order->data_ptr<int>(), (int)N, (int)rows,
+                                             (float)period, starts.data_ptr(), key.data_ptr<int>(), edge->data_ptr<int>(), st));
+        } else {
+            check(mg_painn_grid_rows(fp(r_ij), E, (int)rows, (float)period, key.data_ptr<int>(), st));
+        }
+        auto [by_row, sorted] = sort_values_by_key(key, edge, rows);
         check(mg_segment_row_ptr(sorted.data_ptr<int>(), 0, E, (int)rows, ptr.data_ptr<int>(), st));
         check(mg_painn_grid_table_grad(by_row.data_ptr<int>(), ptr.data_ptr<int>(), src.data_ptr<int>(), dst.data_ptr<int>(), (int)N, E,
                                        fp(r_ij), (int)rows, (float)period, (float)epsilon, fp(g_v), fp(g_a), fp(actv_sliced), fp(v),

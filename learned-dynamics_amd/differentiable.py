@@ -764,7 +764,7 @@ class _PainnGridMessage(torch.autograd.Function):
             grads = ops.painn_grid_message_bwd(table, actv, actv if actv_s is None else actv_s, v, r_ij, g_v.contiguous(),
                                                g_a.contiguous(), graph.src32, graph.dst32, by_dst.row_ptr, by_dst.perm,
                                                getattr(graph, "cell_order", None), ctx.period, ctx.epsilon, need[0], need[1],
-                                               need[2])
+                                               need[2], graph.row_ptr)
             return (*grads, None, None, None, None)
         d = torch.linalg.vector_norm(r_ij, dim=-1).contiguous()
         want = (bool(need[0]), bool(need[1]), bool(need[2]), False)

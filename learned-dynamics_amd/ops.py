@@ -1198,7 +1198,16 @@ mlp_silu_bwd = _ext.mlp_silu_bwd
 painn_edge_encode_fwd = _ext.edge_encode_fwd
 painn_edge_encode_bwd = _ext.edge_encode_bwd
 painn_combine_dual_bwd = _ext.combine_dual_bwd
-painn_grid_message_bwd = _ext.painn_grid_message_bwd
+
+
+def painn_grid_message_bwd(table, actv, actv_sliced, v, r_ij, g_v, g_a, src, dst, row_ptr, order, node_order, period, epsilon,
+                           want_table, want_actv, want_v, src_row_ptr=None):
+    """(d_table, d_actv, d_v) of the message interpolated from its grid.  src_row_ptr: rows of the edges by source; with node_order
+    the grid's gradient then takes the edges in that order of their sources."""
+    return _ext.painn_grid_message_bwd(table, actv, actv_sliced, v, r_ij, g_v, g_a, src, dst, row_ptr, order, node_order, period,
+                                       epsilon, bool(want_table), bool(want_actv), bool(want_v), src_row_ptr)
+
+
 painn_update_train_fwd = _ext.painn_update_train_fwd
 painn_update_train_bwd = _ext.painn_update_train_bwd
 

@@ -1174,3 +1174,49 @@ def test_bias_gradient_of_values_beside_an_infinite_tangent(pkg, R):
     got, = torch.autograd.grad((y, y_t), params[-1:], (g, g_t))
     want = g.double().sum(0)
     assert float((got.double() - want).abs().max() / want.abs().max()) <= 8 * R ** 0.5 * 2 ** -24
+
+
+@pytest.mark.parametrize("N,E,extra", [(1, 7, 0), (255, 40, 0), (257, 3000, 13), (5000, 60000, 0), (70000, 9000, 300)])
+def test_grid_gradient_with_the_edges_in_the_order_of_the_nodes(pkg, ops, N, E, extra):
+    """Every edge once, source by source in any order of the nodes (nodes without edges, more nodes than one block of the scan,
+    edges behind the last row): what reaches the grid is the sum as without an order, up to the order of its terms."""
+    L = importlib.import_module("learned-dynamics_amd._lib")
+    import ctypes
+    gen = torch.Generator().manual_seed(0x947 + N)
+    n, rows, period = 16, 64, 10.0
+    src = torch.sort(torch.randint(0, N, (E,), generator=gen)).values.cuda().int()
+    row_ptr = ops.segment_row_ptr(src, N)
+    order = torch.randperm(N, generator=gen).cuda().int()
+    total = E + extra
+    r = 2 * torch.randn(total, 3, generator=gen).cuda()
+    lib, p = L.load(), lambda t: ctypes.c_void_p(t.data_ptr())
+    key, plain, edge = (torch.full((total,), -1, dtype=torch.int32, device="cuda") for _ in range(3))
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    size = ctypes.c_size_t(0)
+    L.check(lib.mg_painn_grid_rows_by_node_workspace_bytes(N, ctypes.byref(size)))
+    ws = torch.empty(size.value, dtype=torch.uint8, device="cuda")
+    L.check(lib.mg_painn_grid_rows_by_node(p(r), total, p(row_ptr), p(order), N, rows, period, p(ws), p(key), p(edge), stream))
+    L.check(lib.mg_painn_grid_rows(p(r), total, rows, period, p(plain), stream))
+    degree = (row_ptr[1:] - row_ptr[:-1]).long()
+    want = torch.cat([torch.repeat_interleave(row_ptr[:-1].long()[order.long()], degree[order.long()]) + _within(degree[order.long()]),
+                      torch.arange(E, total, device="cuda")])
+    assert torch.equal(edge.long(), want) and torch.equal(key, plain[want])
+    if extra:
+        return
+    rnd = lambda *shape: torch.randn(*shape, generator=gen).cuda()
+    table, actv, v, g_v, g_a = rnd(rows, 4 * n), rnd(N, 4 * n), rnd(N, n, 3), rnd(N, n, 3), rnd(N, n)
+    dst = torch.randint(0, N, (E,), generator=gen).cuda().int()
+    gl = importlib.import_module("learned-dynamics_amd.graph_layers")
+    graph = gl.Graph(src, dst, None, 1, N)
+    args = (table, actv, actv[:, ops.painn_slice_permutation(n, "cuda")].contiguous(), v, r, g_v, g_a, src, dst, graph.by_dst.row_ptr,
+            graph.by_dst.perm)
+    a = ops.painn_grid_message_bwd(*args, order, period, 0.1, True, True, True, src_row_ptr=row_ptr)
+    b = ops.painn_grid_message_bwd(*args, None, period, 0.1, True, True, True)
+    for x, y in zip(a, b):
+        assert float((x - y).abs().max() / y.abs().max()) <= 2 ** -24 * 8 * E ** 0.5
+
+
+def _within(counts):
+    """0 .. c - 1 for every c in turn."""
+    ends = counts.cumsum(0)
+    return torch.arange(int(counts.sum()), device=counts.device) - torch.repeat_interleave(ends - counts, counts)
