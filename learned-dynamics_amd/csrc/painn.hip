@@ -251,11 +251,51 @@ __global__ void __launch_bounds__(256) painn_edge_records_kernel(const float* __
     rec[2 * e + 1] = make_float4(w3, rx * inv, ry * inv, rz * inv);
 }
 
-__global__ void __launch_bounds__(1024) painn_table_message_lds_kernel(
+// The steps of a wave over its nodes' edges, 16 at a time, as scalars: nodes slot, slot + stride, .. of the order; a node without
+// edges is one step without any.  node < 0: past the last.  The rows of the node after the next are requested a node ahead.
+struct NodeSteps {
+    struct Step { int node, b, hi; };
+    const int *row_ptr, *order;
+    long n_nodes, n_edges, slot, stride;
+    Step b;
+    int node_c;
+    __device__ __forceinline__ int node_at(long s) const { return s < n_nodes ? (order ? order[s] : (int)s) : -1; }
+    __device__ __forceinline__ NodeSteps(const int* row_ptr, const int* order, long n_nodes, long n_edges, long slot, long stride)
+        : row_ptr(row_ptr), order(order), n_nodes(n_nodes), n_edges(n_edges), slot(slot), stride(stride) {}
+    __device__ __forceinline__ Step rows_of(int node) const {
+        return node < 0 ? Step{-1, 0, 0} : Step{node, max(row_ptr[node], 0), (int)min((long)row_ptr[node + 1], n_edges)};
+    }
+    __device__ __forceinline__ Step first() {
+        b = rows_of(node_at(slot + stride));
+        node_c = node_at(slot + 2 * stride);
+        return rows_of(node_at(slot));
+    }
+    __device__ __forceinline__ Step next(const Step& s) {
+        if (s.b + 16 < s.hi) return Step{s.node, s.b + 16, s.hi};
+        const Step r = b;
+        slot += stride;
+        b = rows_of(node_c);
+        node_c = node_at(slot + 2 * stride);
+        return r;
+    }
+};
+
+// without edges: the residuals
+__global__ void __launch_bounds__(256) painn_no_edges_kernel(long count, const float* __restrict__ res, float* __restrict__ out) {
+    for (long t = (long)blockIdx.x * 256 + threadIdx.x; t < count; t += (long)gridDim.x * 256) out[t] = res ? res[t] : 0.f;
+}
+
+// Twelve waves on a CU: the rows of the next 16 edges and the indices of those after them are on their way while a step is computed,
+// which takes 140 registers.  16 384 nodes, 1.6 M edges, n = 128: 410 -> 360 us; before, sixteen waves without it (a node's first rows,
+// records and indices were three waits in a row).  In 128 registers 30 of them spill; eight waves 409 us; all four
+// blocks of the filter read ahead 373 us.  What is left: 5.7 GB of gathers at the 20 TB/s of such rows from the L2 (285 us), vector
+// issue (0.22 ms at 2.4 GHz), LDS reads with their conflicts (0.18 ms).
+constexpr int kTableThreads = 768;
+__global__ void __launch_bounds__(kTableThreads) painn_table_message_lds_kernel(
     const int* __restrict__ row_ptr, const int* __restrict__ dst, const int* __restrict__ node_order, long n_nodes,
     const float4* __restrict__ rec, const float* __restrict__ table, int tab_rows, const float* __restrict__ actv_s,
     const float* __restrict__ x_v, int n, const float* __restrict__ res_a, const float* __restrict__ res_v,
-    float* __restrict__ out_a, float* __restrict__ out_v) {
+    float* __restrict__ out_a, float* __restrict__ out_v, long n_edges) {
     extern __shared__ float tab[];                            // (tab_rows + 3) x kSliceRowF
     const int n_slices = n / kSliceChan;
     // consecutive workgroup ids go to consecutive XCDs: with 8 slices every XCD works on one slice, and its L2 only
@@ -268,9 +308,8 @@ __global__ void __launch_bounds__(1024) painn_table_message_lds_kernel(
             ld4(table + (long)(row & (tab_rows - 1)) * 4 * n + k * n + slice * kSliceChan + 4 * c4));
     }
     __syncthreads();
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, waves = blockDim.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), waves = blockDim.x / kWave;
     const int l4 = lane & 3, sub = lane >> 2;                 // 4 channels of edge `sub` of the step
-    constexpr int kPerIter = kWave / 4;
     // 32-bit element offsets (the host checks that they fit) keep the address arithmetic short
     const unsigned a_stride = (unsigned)n_slices * kSliceCols, v_stride = 3u * (unsigned)n;
     const float* a_base = actv_s + slice * kSliceCols + 4 * l4;
@@ -280,59 +319,98 @@ __global__ void __launch_bounds__(1024) painn_table_message_lds_kernel(
     // memory), then the 4 scalar sums
     const bool is_a = sub >= 12;
     const long o_lane = slice * kSliceChan + 4 * l4;
-    for (long slot = (long)group * waves + wave; slot < n_nodes; slot += (long)groups * waves) {
-        const long node = node_order ? node_order[slot] : slot;
-        const int lo = row_ptr[node], hi = row_ptr[node + 1];
-        float acc[16];
+    const float* const res_base = is_a ? (res_a ? res_a + o_lane + (sub - 12) : nullptr) : (res_v ? res_v + o_lane * 3 + sub : nullptr);
+    float* const out_base = is_a ? out_a + o_lane + (sub - 12) : out_v + o_lane * 3 + sub;
+    const long node_stride = is_a ? n : 3L * n;
+
+    NodeSteps steps(row_ptr, node_order, n_nodes, n_edges, (long)group * waves + wave, (long)groups * waves);
+    const unsigned last_node = (unsigned)(n_nodes - 1);
+    struct Edge { float4 a[4], v[3], r0, r1; };
+    float acc[16];
 #pragma unroll
-        for (int k = 0; k < 16; k++) acc[k] = 0.f;
-        int e = lo + sub;
-        unsigned j = 0;
-        float4 ra = make_float4(0.f, 0.f, 0.f, 0.f), rb = ra;
-        if (e < hi) { j = (unsigned)dst[e]; ra = rec[2 * (long)e]; rb = rec[2 * (long)e + 1]; }
-        while (e < hi) {
-            const float* a_row = a_base + j * a_stride;
-            const float* v_row = v_base + j * v_stride;
-            float4 a[4], v[3];
+    for (int k = 0; k < 16; k++) acc[k] = 0.f;
+    // (a slot past the end of its node reads some edge and uses nothing of it)
+    auto edge_of = [&](const NodeSteps::Step& s) { return (unsigned)max(min(s.b + sub, s.hi - 1), 0); };
+    auto row_of = [&](const NodeSteps::Step& s) { return min((unsigned)dst[edge_of(s)], last_node); };
+    auto gather = [&](Edge& d, unsigned e, unsigned j) {
+        const float* a_row = a_base + j * a_stride;
+        const float* v_row = v_base + j * v_stride;
 #pragma unroll
-            for (int k = 0; k < 4; k++) a[k] = ld4(a_row + k * kSliceChan);
+        for (int k = 0; k < 4; k++) d.a[k] = ld4(a_row + k * kSliceChan);
 #pragma unroll
-            for (int k = 0; k < 3; k++) v[k] = ld4(v_row + 4 * k);
-            e += kPerIter;
-            unsigned j_next = 0;
-            float4 na = ra, nb = rb;
-            if (e < hi) { j_next = (unsigned)dst[e]; na = rec[2 * (long)e]; nb = rec[2 * (long)e + 1]; }
-            const float* tp = tab_l + __float_as_int(ra.x);
-            const float w0 = ra.y, w1 = ra.z, w2 = ra.w, w3 = rb.x, ux = rb.y, uy = rb.z, uz = rb.w;
-            float p[4][4];                                    // filter x activation: block k, channel c
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
+        for (int k = 0; k < 3; k++) d.v[k] = ld4(v_row + 4 * k);
+        d.r0 = rec[2 * (long)e];
+        d.r1 = rec[2 * (long)e + 1];
+    };
+    NodeSteps::Step s0 = steps.first(), s1 = steps.next(s0), s2 = steps.next(s1);
+    if (s0.node < 0) return;
+    Edge even, odd;
+    gather(even, edge_of(s0), row_of(s0));
+    unsigned j1 = row_of(s1);
+    // One step: the rows of the next step's edges are requested before this step's are used, the indices of the one after that
+    // behind them.  (No branch around the loads, which would make every wait one for all of them.)
+    auto step = [&](const Edge& d, Edge& d_next) {
+        const bool node_ends = s0.b + 16 >= s0.hi;
+        float res = 0.f;
+        if (node_ends && res_base) res = res_base[s0.node * node_stride];
+        __builtin_amdgcn_sched_barrier(0);
+        gather(d_next, edge_of(s1), j1);
+        j1 = row_of(s2);
+        __builtin_amdgcn_sched_barrier(0);
+        if (s0.b + sub < s0.hi) {
+            const float* tp = tab_l + __float_as_int(d.r0.x);
+            const float w0 = d.r0.y, w1 = d.r0.z, w2 = d.r0.w, w3 = d.r1.x, ux = d.r1.y, uy = d.r1.z, uz = d.r1.w;
+            const float vv[12] = {d.v[0].x, d.v[0].y, d.v[0].z, d.v[0].w, d.v[1].x, d.v[1].y, d.v[1].z, d.v[1].w,
+                                  d.v[2].x, d.v[2].y, d.v[2].z, d.v[2].w};
+            // filter x activation, block k; one block at a time: the registers of the four grid rows are used again
+            auto filtered = [&](int k, float (&p)[4]) {
+                __builtin_amdgcn_sched_barrier(0);
                 const float4 t0 = ld4(tp + k * kSliceChan), t1 = ld4(tp + kSliceRowF + k * kSliceChan),
                              t2 = ld4(tp + 2 * kSliceRowF + k * kSliceChan), t3 = ld4(tp + 3 * kSliceRowF + k * kSliceChan);
-                p[k][0] = (w0 * t0.x + w1 * t1.x + w2 * t2.x + w3 * t3.x) * a[k].x;
-                p[k][1] = (w0 * t0.y + w1 * t1.y + w2 * t2.y + w3 * t3.y) * a[k].y;
-                p[k][2] = (w0 * t0.z + w1 * t1.z + w2 * t2.z + w3 * t3.z) * a[k].z;
-                p[k][3] = (w0 * t0.w + w1 * t1.w + w2 * t2.w + w3 * t3.w) * a[k].w;
-            }
-            const float vv[12] = {v[0].x, v[0].y, v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w,
-                                  v[2].x, v[2].y, v[2].z, v[2].w};
+                p[0] = (w0 * t0.x + w1 * t1.x + w2 * t2.x + w3 * t3.x) * d.a[k].x;
+                p[1] = (w0 * t0.y + w1 * t1.y + w2 * t2.y + w3 * t3.y) * d.a[k].y;
+                p[2] = (w0 * t0.z + w1 * t1.z + w2 * t2.z + w3 * t3.z) * d.a[k].z;
+                p[3] = (w0 * t0.w + w1 * t1.w + w2 * t2.w + w3 * t3.w) * d.a[k].w;
+            };
+            float p[4];
+            filtered(0, p);
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+#pragma unroll
+                for (int i = 0; i < 3; i++) acc[3 * c + i] = fmaf(vv[3 * c + i], p[c], acc[3 * c + i]);
+            filtered(1, p);
 #pragma unroll
             for (int c = 0; c < 4; c++) {
                 const float x = vv[3 * c], y = vv[3 * c + 1], z = vv[3 * c + 2];
-                const float cx = y * uz - z * uy, cy = z * ux - x * uz, cz = x * uy - y * ux;   // v x u
-                acc[3 * c + 0] = fmaf(ux, p[2][c], fmaf(cx, p[1][c], fmaf(x, p[0][c], acc[3 * c + 0])));
-                acc[3 * c + 1] = fmaf(uy, p[2][c], fmaf(cy, p[1][c], fmaf(y, p[0][c], acc[3 * c + 1])));
-                acc[3 * c + 2] = fmaf(uz, p[2][c], fmaf(cz, p[1][c], fmaf(z, p[0][c], acc[3 * c + 2])));
-                acc[12 + c] += p[3][c];
+                acc[3 * c + 0] = fmaf(y * uz - z * uy, p[c], acc[3 * c + 0]);                 // v x u
+                acc[3 * c + 1] = fmaf(z * ux - x * uz, p[c], acc[3 * c + 1]);
+                acc[3 * c + 2] = fmaf(x * uy - y * ux, p[c], acc[3 * c + 2]);
             }
-            j = j_next; ra = na; rb = nb;
+            filtered(2, p);
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                acc[3 * c + 0] = fmaf(ux, p[c], acc[3 * c + 0]);
+                acc[3 * c + 1] = fmaf(uy, p[c], acc[3 * c + 1]);
+                acc[3 * c + 2] = fmaf(uz, p[c], acc[3 * c + 2]);
+            }
+            filtered(3, p);
+#pragma unroll
+            for (int c = 0; c < 4; c++) acc[12 + c] += p[c];
         }
-        const long o = node * n + o_lane;
-        float sum = sum_over_slots(acc, lane);
-        float* outp = is_a ? out_a + o + (sub - 12) : out_v + o * 3 + sub;
-        const float* resp = is_a ? (res_a ? res_a + o + (sub - 12) : nullptr) : (res_v ? res_v + o * 3 + sub : nullptr);
-        if (resp) sum += *resp;
-        *outp = sum;
+        if (node_ends) {
+            out_base[s0.node * node_stride] = sum_over_slots(acc, lane) + res;
+#pragma unroll
+            for (int k = 0; k < 16; k++) acc[k] = 0.f;
+        }
+        s0 = s1;
+        s1 = s2;
+        s2 = steps.next(s2);
+    };
+    while (true) {
+        step(even, odd);
+        if (s0.node < 0) return;
+        step(odd, even);
+        if (s0.node < 0) return;
     }
 }
 
@@ -599,6 +677,11 @@ int mg_painn_table_message_sliced(const int* row_ptr, const int* dst, const int*
                "mg_painn_table_message_sliced: n must be a multiple of %d and the operands 16-byte aligned", kSliceChan);
     MG_REQUIRE((long)n_nodes * 4 * n < (1L << 32), "mg_painn_table_message_sliced: n_nodes * 4 n must be below 2^32");
     MG_REQUIRE(n_edges < (1L << 31), "mg_painn_table_message_sliced: n_edges must be below 2^31");
+    if (n_edges == 0) {
+        hipLaunchKernelGGL(painn_no_edges_kernel, dim3(256), dim3(256), 0, (hipStream_t)stream, (long)n_nodes * n, res_a, out_a);
+        hipLaunchKernelGGL(painn_no_edges_kernel, dim3(256), dim3(256), 0, (hipStream_t)stream, 3L * n_nodes * n, res_v, out_v);
+        return check_launch("mg_painn_table_message_sliced");
+    }
     const int n_slices = n / kSliceChan;
     const size_t lds_bytes = (size_t)(table_rows + kSliceExtraRows) * kSliceRowF * sizeof(float);
     // more than 64 KB of dynamic LDS has to be asked for (per device, so on every call)
@@ -608,10 +691,10 @@ int mg_painn_table_message_sliced(const int* row_ptr, const int* dst, const int*
     long groups = ceil_div(256, n_slices);                    // one workgroup per CU
     const long max_groups = ceil_div(n_nodes, 16);
     if (groups > max_groups) groups = max_groups;
-    hipLaunchKernelGGL(painn_table_message_lds_kernel, dim3((unsigned)(groups * n_slices)), dim3(1024), lds_bytes,
+    hipLaunchKernelGGL(painn_table_message_lds_kernel, dim3((unsigned)(groups * n_slices)), dim3(kTableThreads), lds_bytes,
                        (hipStream_t)stream, row_ptr, dst, node_order, (long)n_nodes,
                        reinterpret_cast<const float4*>(records), table, table_rows, actv_sliced, x_v, n, res_a, res_v,
-                       out_a, out_v);
+                       out_a, out_v, n_edges);
     return check_launch("mg_painn_table_message_sliced");
 }
 

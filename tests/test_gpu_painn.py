@@ -654,3 +654,29 @@ def test_submodules_are_called_where_a_call_is_more_than_their_parameters(pkg, h
         grads = [torch.autograd.grad((a ** 2).sum() + (v ** 2).sum(), (x_a, x_v)) for a, v in ((got_a, got_v), (want_a, want_v))]
         for a, b in zip(*grads):
             torch.testing.assert_close(a, b, rtol=0, atol=2e-5 * float(b.abs().max()))
+
+
+@pytest.mark.parametrize("degrees", [(0,), (0, 0, 1), (16, 0, 15, 17, 0, 33, 32, 1), (0, 100, 0), tuple(range(0, 70)) * 12, (48,) * 1000])
+@pytest.mark.parametrize("ordered", [False, True])
+def test_message_with_the_grid_in_lds_over_nodes_of_any_degree(pkg, degrees, ordered):
+    """Nodes without edges, with whole and partial steps of 16, fewer and more nodes than waves, edges behind the last row that hold
+    no node (a capacity-sized graph), rows that hold infinities and belong to no edge: against the kernel that reads the grid from
+    memory.  Both add a node's edges in fp32, in different order: 8 2^-24 sqrt(degree) of the largest entry, and the place of an
+    edge between grid rows, each kernel's own, carries rows 2^-24."""
+    ops = importlib.import_module("learned-dynamics_amd.ops")
+    gen = torch.Generator().manual_seed(len(degrees))
+    n, rows, N, period = 32, 64, len(degrees) + 1, 10.0
+    row_ptr = torch.cat([torch.zeros(1, dtype=torch.int64), torch.tensor(degrees + (0,)).cumsum(0)]).int().cuda()
+    E = int(row_ptr[-1])
+    dst = torch.cat([torch.randint(0, N - 1, (E,), generator=gen), torch.full((5,), 2 ** 31 - 1)]).int().cuda()
+    r = torch.randn(E + 5, 3, generator=gen).cuda() * 2
+    table, actv, v = (torch.randn(*s, generator=gen).cuda() for s in ((rows, 4 * n), (N, 4 * n), (N, n, 3)))
+    actv[N - 1], v[N - 1] = float("inf"), float("nan")
+    res_a, res_v = torch.randn(N, n, generator=gen).cuda(), torch.randn(N, n, 3, generator=gen).cuda()
+    order = torch.randperm(N, generator=gen).int().cuda() if ordered else None
+    perm = ops.painn_slice_permutation(n, "cuda")
+    for res in ((None, None), (res_a, res_v)):
+        a, b = ops.painn_table_message_sliced(row_ptr, dst, r, table, period, actv[:, perm].contiguous(), v, 0.1, *res, node_order=order)
+        want_a, want_b = ops.painn_table_message(row_ptr, dst, r, table, period, actv, v, 0.1, *res)
+        for x, y in ((a, want_a), (b, want_b)):
+            assert float((x - y).abs().max()) <= 2 ** -24 * (8 * max(1, max(degrees)) ** 0.5 + rows) * max(1.0, float(y.abs().max()))
