@@ -31,6 +31,7 @@
 //   when box/cutoff is not an integer the cells are narrower than the cutoff and
 //   pairs two cells apart are not listed.
 #include "common.hpp"
+#include <type_traits>
 #include <mutex>
 #include <type_traits>
 
@@ -413,19 +414,25 @@ __device__ __forceinline__ int block_excl_scan(int v, int* total, int* lds /* >=
     return off + incl - v;
 }
 
-__global__ void __launch_bounds__(kScanThreads) scan_sums_kernel(const int* __restrict__ in, long n,
-                                                                 int* block_sums, int* block_max) {
+// sums and maxima per tile; scanned (or null, or `in` itself): the sums inside the tile up to and with each entry
+__global__ void __launch_bounds__(kScanThreads) scan_sums_kernel(const int* in, long n, int* block_sums, int* block_max, int* scanned) {
     __shared__ int lds[8];
     const long base = (long)blockIdx.x * kScanTile + (long)threadIdx.x * kScanItems;
-    int s = 0, m = 0;
+    int s = 0, m = 0, item[kScanItems];
 #pragma unroll
     for (int k = 0; k < kScanItems; k++) {
-        const int v = (base + k < n) ? in[base + k] : 0;
-        s += v;
-        m = v > m ? v : m;
+        item[k] = (base + k < n) ? in[base + k] : 0;
+        s += item[k];
+        m = item[k] > m ? item[k] : m;
     }
     int total;
-    block_excl_scan(s, &total, lds);
+    int sum = block_excl_scan(s, &total, lds);
+    if (scanned)
+#pragma unroll
+        for (int k = 0; k < kScanItems; k++) {
+            sum += item[k];
+            if (base + k < n) scanned[base + k] = sum;
+        }
     // block max through the same LDS words
     for (int d = kWave / 2; d > 0; d >>= 1) { int t = __shfl_xor(m, d); m = t > m ? t : m; }
     if ((threadIdx.x & (kWave - 1)) == 0) lds[threadIdx.x / kWave] = m;
@@ -744,6 +751,10 @@ struct EdgeOut {
     float* r_ij;        // or null
     const float* x;     // unwrapped positions (with r_ij)
 
+    // the arrays from edge e on
+    __device__ __forceinline__ EdgeOut from(int e) const {
+        return EdgeOut{src + e, dst + e, src64 ? src64 + e : nullptr, dst64 ? dst64 + e : nullptr, r_ij ? r_ij + 3 * (long)e : nullptr, x};
+    }
     __device__ __forceinline__ void store(int e, int i, int j) const {
         src[e] = i;
         dst[e] = j;
@@ -1018,35 +1029,40 @@ __global__ void __launch_bounds__(kBoxThreads) box_search_kernel(const float* __
 // rows and the sums of the tiles before (tiled: scan_sums_kernel has left them), or simply all of them (at most
 // kDirectRows degrees from the L2: cheaper than a launch).  Workgroup 0 also reduces everything to the statistics.  The
 // edge's int64 indices and its vector are written here, where i and j are in registers, instead of by three kernels that
-// read the edge list back.  Bound by the stores, 36 bytes per edge with everything asked for, once a thread has several
-// edges' loads in flight: kFillUnroll edges at a time, rows found without branches.
+// read the edge list back.  A wave takes RW rows, a lane an edge of each: what a row's edges are does not depend on where they go,
+// so that its hits, its atom and the degrees of the rows before it are all requested at once, and the neighbours' atoms as
+// soon as the hits are there.  6.8 M edges: 83 us (97 with the edges of 64 rows dealt out to the threads, whose rows had to be found,
+// and a barrier after the sums).  Bound by the stores, 36 bytes per edge with everything asked for (44 us of them, 243 MB), and
+// the two dependent loads before them, which wait behind the stores of other waves; 16-byte stores of four edges to a thread
+// and eight waves per SIMD changed nothing or spilled.
 constexpr long kDirectRows = 16384;
-constexpr int kFillUnroll = 4;
-template <typename HitT>
-__global__ void __launch_bounds__(256) graph_fill_kernel(Grid g, Workspace w, int rows_per, int tiled, int n_box,
-                                                         int* __restrict__ row_ptr, int* __restrict__ edge_counts,
-                                                         int* stats, int capacity, EdgeOut out, int* __restrict__ order) {
-    __shared__ int rp[kFillRows + 1];
-    __shared__ int first_row[kFillRows];      // first row of the box that the row belongs to
-    __shared__ float3 x_row[kFillRows];
-    __shared__ long long wave_before[4], wave_all[4];
-    __shared__ int wave_mx[4], wave_cell[4], wave_flag[4];
+template <typename HitT, int RW>
+__global__ void __launch_bounds__(256) graph_fill_kernel(Grid g, Workspace w, int tiled, int n_box, int* __restrict__ row_ptr,
+                                                         int* __restrict__ edge_counts, int* stats, int capacity, EdgeOut out,
+                                                         int* __restrict__ order) {
+    constexpr int rows_per = 4 * RW;
+    static_assert(rows_per <= kWave && kScanTile % rows_per == 0, "a wave holds the degrees of all rows, which lie in one tile");
+    __shared__ long long wave_all[4];
+    __shared__ int wave_before[4], wave_mx[4], wave_cell[4], wave_flag[4];
     const long A = (long)g.batch * g.nodes;
     const long r0 = (long)blockIdx.x * rows_per;
     const int nrows = A - r0 < rows_per ? (int)(A - r0) : rows_per;
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-    const bool totals = blockIdx.x == 0;
-    const int my_degree = (wave == 0 && lane < nrows) ? w.degree[r0 + lane] : 0;
-    const int tile = tiled ? (int)(r0 / kScanTile) : 0;
-    long long before = 0, all = 0;
-    int mx = 0, cell = 0, flag = 0;
-    if (tiled) {
-        for (int k = tid; k < tile; k += 256) before += w.deg_sums[k];
-        for (long r = (long)tile * kScanTile + tid; r < r0; r += 256) before += w.degree[r];
-    } else {
-        for (long r = tid; r < r0; r += 256) before += w.degree[r];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int cap = w.hit_cap;
+    const HitT* __restrict__ hits = static_cast<const HitT*>(w.hits);
+    const float* __restrict__ x = out.x;
+    int hit[RW];
+    float3 xi[RW];
+#pragma unroll
+    for (int k = 0; k < RW; k++) {                    // (a wave's rows are scalars: so are their addresses)
+        const int at = wave * RW + k;
+        const long r = r0 + (at < nrows ? at : 0);
+        hit[k] = lane < cap ? (int)hits[r * cap + lane] : 0;     // (past the row's degree: not used)
+        if (x) xi[k] = load3(x + 3 * r);
     }
-    if (totals) {
+    if (blockIdx.x == 0) {                                        // the statistics of the whole graph: the host waits for them
+        long long all = 0;
+        int mx = 0, cell = 0, flag = 0;
         const long n = tiled ? A / kScanTile + 1 : A;             // ceil((A + 1) / kScanTile) tiles
         const int* sums = tiled ? w.deg_sums : w.degree;
         const int* maxima = tiled ? w.deg_max : w.degree;
@@ -1060,10 +1076,7 @@ __global__ void __launch_bounds__(256) graph_fill_kernel(Grid g, Workspace w, in
             cell = v > cell ? v : cell;
             flag |= w.box_max[k] & kNanBit;
         }
-    }
-    for (int d = kWave / 2; d > 0; d >>= 1) {
-        before += __shfl_xor(before, d);
-        if (totals) {
+        for (int d = kWave / 2; d > 0; d >>= 1) {
             all += __shfl_xor(all, d);
             int t = __shfl_xor(mx, d);
             mx = t > mx ? t : mx;
@@ -1071,91 +1084,95 @@ __global__ void __launch_bounds__(256) graph_fill_kernel(Grid g, Workspace w, in
             cell = t > cell ? t : cell;
             flag |= __shfl_xor(flag, d);
         }
-    }
-    if (lane == 0) {
-        wave_before[wave] = before;
-        wave_all[wave] = all;
-        wave_mx[wave] = mx;
-        wave_cell[wave] = cell;
-        wave_flag[wave] = flag;
-    }
-    __syncthreads();
-    if (totals && tid == 0) {
-        for (int k = 1; k < 4; k++) {
-            all += wave_all[k];
-            mx = wave_mx[k] > mx ? wave_mx[k] : mx;
-            cell = wave_cell[k] > cell ? wave_cell[k] : cell;
-            flag |= wave_flag[k];
+        if (lane == 0) {
+            wave_all[wave] = all;
+            wave_mx[wave] = mx;
+            wave_cell[wave] = cell;
+            wave_flag[wave] = flag;
         }
-        // (a host may be polling these words: each is stored once, at system scope)
-        const int words[4] = {all > 0x7fffffffLL ? 0x7fffffff : (int)all, cell, mx,
-                              (all > 0x7fffffffLL ? 1 : 0) | (flag ? 4 : 0)};
-#pragma unroll
-        for (int k = 0; k < 4; k++) __hip_atomic_store(stats + k, words[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    if (wave == 0) {
-        const int first = (int)(wave_before[0] + wave_before[1] + wave_before[2] + wave_before[3]);
-        const int incl = wave_incl_scan(my_degree, lane);
-        if (lane < nrows) {
-            rp[lane + 1] = first + incl;
-            row_ptr[r0 + lane] = first + incl - my_degree;
-            const long next = r0 + lane + 1;
-            if (next == A) row_ptr[A] = first + incl;
-            const unsigned q = (unsigned)next / (unsigned)g.nodes;                // (next < 2^31: 32-bit divide)
-            if (q * (unsigned)g.nodes == (unsigned)next) edge_counts[q - 1] = first + incl;
-        }
-        if (lane == 0) rp[0] = first;
-    }
-    if (wave == 0 && lane >= nrows && lane < rows_per) rp[lane + 1] = 0x7fffffff;
-    if (wave == 1 && lane < nrows) {
-        const unsigned k = (unsigned)(r0 + lane);
-        const int first = (int)(k / (unsigned)g.nodes) * g.nodes;
-        first_row[lane] = first;
-        if (order) order[k] = first + __float_as_int(w.sorted[k].w);
-    }
-    if (wave == 2 && lane < nrows && out.r_ij) x_row[lane] = load3(out.x + 3 * (r0 + lane));
-    __syncthreads();
-    const int cap = w.hit_cap;
-    const HitT* __restrict__ hits = static_cast<const HitT*>(w.hits);
-    const int e_hi = rp[nrows];
-    const Box3 box = box_of(g.bx, g.by, g.bz);
-    for (int e0 = rp[0] + tid; e0 < e_hi; e0 += 256 * kFillUnroll) {
-        int row[kFillUnroll], j[kFillUnroll];
-        bool ok[kFillUnroll];
-#pragma unroll
-        for (int u = 0; u < kFillUnroll; u++) {
-            const int e = e0 + 256 * u;
-            int lo = 0;                                // last row with rp <= e (rp ends in INT_MAX past the last row)
-            for (int step = rows_per >> 1; step > 0; step >>= 1) lo += rp[lo + step] <= e ? step : 0;
-            lo = lo < nrows ? lo : nrows - 1;          // (a position past the last edge: discarded below, but it must not
-                                                       // name a row that is not staged, its atom is read all the same)
-            const int idx = e - rp[lo], deg = rp[lo + 1] - rp[lo];
-            ok[u] = e < e_hi && deg <= cap && idx >= 0 && idx < deg && e >= 0 && e < capacity;
-            row[u] = lo;
-            j[u] = ok[u] ? (int)hits[(r0 + lo) * cap + idx] : 0;
-        }
-        float3 xj[kFillUnroll];
-#pragma unroll
-        for (int u = 0; u < kFillUnroll; u++) {
-            j[u] += first_row[row[u]];
-            if (out.r_ij) xj[u] = load3(out.x + 3 * (long)j[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < kFillUnroll; u++)
-            if (ok[u]) out.store(e0 + 256 * u, (int)r0 + row[u], j[u]);
-        if (out.r_ij) {
-#pragma unroll
-            for (int u = 0; u < kFillUnroll; u++) {
-                const float3 r = wrapped_difference(xj[u], x_row[row[u]], box);
-                if (ok[u]) out.store_vector(e0 + 256 * u, r);
+        __syncthreads();
+        if (tid == 0) {
+            for (int k = 1; k < 4; k++) {
+                all += wave_all[k];
+                mx = wave_mx[k] > mx ? wave_mx[k] : mx;
+                cell = wave_cell[k] > cell ? wave_cell[k] : cell;
+                flag |= wave_flag[k];
             }
+            // (a host may be polling these words: each is stored once, at system scope)
+            const int words[4] = {all > 0x7fffffffLL ? 0x7fffffff : (int)all, cell, mx,
+                                  (all > 0x7fffffffLL ? 1 : 0) | (flag ? 4 : 0)};
+#pragma unroll
+            for (int k = 0; k < 4; k++) __hip_atomic_store(stats + k, words[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
-    for (int r = wave; r < nrows; r += 4)
-        if (rp[r + 1] - rp[r] > cap) refill_row(g, w, (int)(r0 + r), rp[r], capacity, out);
+    // of row r0 + lane
+    int my_degree, my_start;
+    if (tiled) {
+        // (scan_sums_kernel has left the sums inside the tile in the place of the degrees; a wave adds the tiles before by itself)
+        const int tile = (int)(r0 / kScanTile);
+        int incl = 0, prev = 0, before = 0;
+        if (lane < nrows) {
+            incl = w.degree[r0 + lane];
+            if ((r0 + lane) % kScanTile != 0) prev = w.degree[r0 + lane - 1];
+        }
+        for (int k = lane; k < tile; k += kWave) before += w.deg_sums[k];
+        for (int d = kWave / 2; d > 0; d >>= 1) before += __shfl_xor(before, d);
+        my_degree = incl - prev;
+        my_start = before + prev;
+    } else {
+        my_degree = lane < nrows ? w.degree[r0 + lane] : 0;
+        int before = 0;
+        for (long r = tid; r < r0; r += 256) before += w.degree[r];
+        for (int d = kWave / 2; d > 0; d >>= 1) before += __shfl_xor(before, d);
+        if (lane == 0) wave_before[wave] = before;
+        const int incl = wave_incl_scan(my_degree, lane);         // (every wave by itself)
+        __syncthreads();
+        my_start = wave_before[0] + wave_before[1] + wave_before[2] + wave_before[3] + incl - my_degree;
+    }
+
+    const int my_box = (int)((unsigned)(r0 + (lane < nrows ? lane : 0)) / (unsigned)g.nodes) * g.nodes;      // first row of the row's box
+    float3 xj[RW];
+#pragma unroll
+    for (int k = 0; k < RW; k++) {
+        const int at = wave * RW + k, degree = __builtin_amdgcn_readlane(my_degree, at);
+        hit[k] = lane < degree ? __builtin_amdgcn_readlane(my_box, at) + hit[k] : (int)r0;
+        if (x) xj[k] = load3(x + 3 * (long)(degree <= cap ? hit[k] : (int)r0));
+    }
+    const Box3 box = box_of(g.bx, g.by, g.bz);
+#pragma unroll
+    for (int k = 0; k < RW; k++) {
+        const int at = wave * RW + k, degree = __builtin_amdgcn_readlane(my_degree, at), start = __builtin_amdgcn_readlane(my_start, at);
+        if (at >= nrows || start < 0) continue;
+        const int row = (int)r0 + at;
+        if (degree > cap) {
+            refill_row(g, w, row, start, capacity, out);
+            continue;
+        }
+        const EdgeOut here = out.from(start);
+        const int room = capacity - start, n = degree < room ? degree : room;
+        if (lane < n) {
+            here.store(lane, row, hit[k]);
+            if (x) here.store_vector(lane, wrapped_difference(xj[k], xi[k], box));
+        }
+        for (int t = lane + kWave; t < n; t += kWave) {
+            const int j = __builtin_amdgcn_readlane(my_box, at) + (int)hits[(long)row * cap + t];
+            here.store(t, row, j);
+            if (x) here.store_vector(t, wrapped_difference(load3(x + 3 * (long)j), xi[k], box));
+        }
+    }
+    if (wave == 0 && lane < nrows) {
+        row_ptr[r0 + lane] = my_start;
+        const long next = r0 + lane + 1;
+        if (next == A) row_ptr[A] = my_start + my_degree;
+        const unsigned q = (unsigned)next / (unsigned)g.nodes;                    // (next < 2^31: 32-bit divide)
+        if (q * (unsigned)g.nodes == (unsigned)next) edge_counts[q - 1] = my_start + my_degree;
+    }
+    if (wave == 1 && lane < nrows && order) {
+        const unsigned k = (unsigned)(r0 + lane);
+        order[k] = (int)(k / (unsigned)g.nodes) * g.nodes + __float_as_int(w.sorted[k].w);
+    }
 }
 
-// order[k] = global id of the k-th atom in cell order (cells x-major, atoms by id inside a cell)
 __global__ void __launch_bounds__(256) cell_order_kernel(Grid g, Workspace w, int* __restrict__ order) {
     const long A = (long)g.batch * g.nodes;
     const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1248,7 +1265,7 @@ int run_scan(const int* in, long n, int* out, Workspace& w, int* out_total, int*
         return check_launch("neighbour scan");
     }
     const int nblocks = (int)ceil_div(n + 1, kScanTile);
-    hipLaunchKernelGGL(scan_sums_kernel, dim3(nblocks), dim3(kScanThreads), 0, st, in, n, w.block_sums, w.block_max);
+    hipLaunchKernelGGL(scan_sums_kernel, dim3(nblocks), dim3(kScanThreads), 0, st, in, n, w.block_sums, w.block_max, (int*)nullptr);
     hipLaunchKernelGGL(scan_apply_kernel, dim3(nblocks), dim3(kScanThreads), 0, st, in, n, w.block_sums, w.block_max,
                        nblocks, out, nodes, edge_counts, out_total, out_max, out_overflow, (const int*)nullptr, 0,
                        (int*)nullptr);
@@ -1417,7 +1434,7 @@ int mg_neighbour_count(const float* x, int batch, int nodes, float cutoff, float
     const int deg_tiles = (int)ceil_div(A + 1, kScanTile);
     if (int s = enqueue_search(x, g, w, st)) return s;
     hipLaunchKernelGGL(scan_sums_kernel, dim3((unsigned)deg_tiles), dim3(kScanThreads), 0, st, (const int*)w.degree, A,
-                       w.deg_sums, w.deg_max);
+                       w.deg_sums, w.deg_max, (int*)nullptr);
     hipLaunchKernelGGL(scan_apply_kernel, dim3((unsigned)deg_tiles), dim3(kScanThreads), 0, st, (const int*)w.degree, A,
                        (const int*)w.deg_sums, (const int*)w.deg_max, deg_tiles, row_ptr, nodes, edge_counts, stats + 0,
                        stats + 2, stats + 3, (const int*)w.box_max, box_max_entries(g), stats + 1);
@@ -1465,7 +1482,7 @@ int mg_graph_search(const float* x, int batch, int nodes, float cutoff, float bo
     const long A = (long)batch * nodes;
     if (A > kDirectRows)
         hipLaunchKernelGGL(scan_sums_kernel, dim3((unsigned)ceil_div(A + 1, kScanTile)), dim3(kScanThreads), 0, st,
-                           (const int*)w.degree, A, w.deg_sums, w.deg_max);
+                           (const int*)w.degree, A, w.deg_sums, w.deg_max, w.degree);
     return check_launch("mg_graph_search");
 }
 
@@ -1490,17 +1507,20 @@ int mg_graph_fill(const float* x, const void* workspace, size_t workspace_bytes,
     size_t needed = 0;
     if (workspace_bytes == 0 || !layout(g, base, workspace_bytes, &w, &needed))
         return fail(MG_ERR_WORKSPACE, "mg_graph_fill: workspace has %zu bytes, at least %zu needed", workspace_bytes, needed);
-    const EdgeOut out{src, dst, src64, dst64, r_ij, x};
-    // few rows: workgroups of 8, so that a small graph still spreads over the chip
-    const int rows_per = A <= 4096 ? 8 : kFillRows;
-    const dim3 grid((unsigned)ceil_div(A, rows_per));
+    const EdgeOut out{src, dst, src64, dst64, r_ij, r_ij ? x : nullptr};
     const int tiled = A > kDirectRows ? 1 : 0;
-    if (w.hit_bytes == 2)
-        hipLaunchKernelGGL(graph_fill_kernel<unsigned short>, grid, dim3(256), 0, st, g, w, rows_per, tiled,
-                           box_max_entries(g), row_ptr, edge_counts, stats, capacity, out, order);
-    else
-        hipLaunchKernelGGL(graph_fill_kernel<int>, grid, dim3(256), 0, st, g, w, rows_per, tiled, box_max_entries(g), row_ptr,
-                           edge_counts, stats, capacity, out, order);
+    // Few rows: one to a wave, so that a small graph still spreads over the chip (337 atoms: 4.3 us, 9 with eight); otherwise eight, whose
+    // loads are in flight together (131 072 rows of 52 edges: one 107, four 88, eight 83 us)
+    auto launch = [&](auto hit, auto rw) {
+        hipLaunchKernelGGL((graph_fill_kernel<decltype(hit), decltype(rw)::value>), dim3((unsigned)ceil_div(A, 4 * decltype(rw)::value)),
+                           dim3(256), 0, st, g, w, tiled, box_max_entries(g), row_ptr, edge_counts, stats, capacity, out, order);
+    };
+    auto with_rows = [&](auto hit) {
+        if (A <= 4096) launch(hit, std::integral_constant<int, 1>{});
+        else launch(hit, std::integral_constant<int, 8>{});
+    };
+    if (w.hit_bytes == 2) with_rows((unsigned short)0);
+    else with_rows((int)0);
     return check_launch("mg_graph_fill");
 }
 
