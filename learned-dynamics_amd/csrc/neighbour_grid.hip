@@ -1024,6 +1024,77 @@ __global__ void __launch_bounds__(kBoxThreads) box_search_kernel(const float* __
     }
 }
 
+// The statistics of the whole graph, by the first workgroup before anything else: the host waits for them.
+__device__ void graph_statistics(const Workspace& w, long A, int tiled, int n_box, int* stats) {
+    __shared__ long long wave_all[4];
+    __shared__ int wave_mx[4], wave_cell[4], wave_flag[4];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    long long all = 0;
+    int mx = 0, cell = 0, flag = 0;
+    const long n = tiled ? A / kScanTile + 1 : A;             // ceil((A + 1) / kScanTile) tiles
+    const int* sums = tiled ? w.deg_sums : w.degree;
+    const int* maxima = tiled ? w.deg_max : w.degree;
+    for (long k = tid; k < n; k += 256) {
+        all += sums[k];
+        const int m = maxima[k];
+        mx = m > mx ? m : mx;
+    }
+    for (int k = tid; k < n_box; k += 256) {
+        const int v = w.box_max[k] & ~kNanBit;
+        cell = v > cell ? v : cell;
+        flag |= w.box_max[k] & kNanBit;
+    }
+    for (int d = kWave / 2; d > 0; d >>= 1) {
+        all += __shfl_xor(all, d);
+        int t = __shfl_xor(mx, d);
+        mx = t > mx ? t : mx;
+        t = __shfl_xor(cell, d);
+        cell = t > cell ? t : cell;
+        flag |= __shfl_xor(flag, d);
+    }
+    if (lane == 0) {
+        wave_all[wave] = all;
+        wave_mx[wave] = mx;
+        wave_cell[wave] = cell;
+        wave_flag[wave] = flag;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        for (int k = 1; k < 4; k++) {
+            all += wave_all[k];
+            mx = wave_mx[k] > mx ? wave_mx[k] : mx;
+            cell = wave_cell[k] > cell ? wave_cell[k] : cell;
+            flag |= wave_flag[k];
+        }
+        // (a host may be polling these words: each is stored once, at system scope)
+        const int words[4] = {all > 0x7fffffffLL ? 0x7fffffff : (int)all, cell, mx,
+                              (all > 0x7fffffffLL ? 1 : 0) | (flag ? 4 : 0)};
+#pragma unroll
+        for (int k = 0; k < 4; k++) __hip_atomic_store(stats + k, words[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+// Row r0 + lane where scan_sums_kernel has left the sums inside the tile in the place of the degrees; a wave adds the tiles before by
+// itself.  The rows r0 .. r0 + nrows - 1 lie in one tile.
+struct FillRow { int degree, start; };
+__device__ __forceinline__ FillRow row_of_tile(const Workspace& w, long r0, int lane, int nrows) {
+    const int tile = (int)(r0 / kScanTile);
+    int incl = 0, prev = 0, before = 0;
+    if (lane < nrows) {
+        incl = w.degree[r0 + lane];
+        if ((r0 + lane) % kScanTile != 0) prev = w.degree[r0 + lane - 1];
+    }
+    for (int k = lane; k < tile; k += kWave) before += w.deg_sums[k];
+    for (int d = kWave / 2; d > 0; d >>= 1) before += __shfl_xor(before, d);
+    return FillRow{incl - prev, before + prev};
+}
+__device__ __forceinline__ void put_row(const Grid& g, long A, long r, const FillRow& own, int* row_ptr, int* edge_counts) {
+    row_ptr[r] = own.start;
+    const long next = r + 1;
+    if (next == A) row_ptr[A] = own.start + own.degree;
+    const unsigned q = (unsigned)next / (unsigned)g.nodes;                        // (next < 2^31: 32-bit divide)
+    if (q * (unsigned)g.nodes == (unsigned)next) edge_counts[q - 1] = own.start + own.degree;
+}
+
 // Row pointer, statistics and edges of a whole graph in one kernel.  A workgroup takes `rows_per` consecutive rows and
 // finds the position of its first edge by adding up the degrees of the rows before it: those of its tile of kScanTile
 // rows and the sums of the tiles before (tiled: scan_sums_kernel has left them), or simply all of them (at most
@@ -1042,8 +1113,7 @@ __global__ void __launch_bounds__(256) graph_fill_kernel(Grid g, Workspace w, in
                                                          int* __restrict__ order) {
     constexpr int rows_per = 4 * RW;
     static_assert(rows_per <= kWave && kScanTile % rows_per == 0, "a wave holds the degrees of all rows, which lie in one tile");
-    __shared__ long long wave_all[4];
-    __shared__ int wave_before[4], wave_mx[4], wave_cell[4], wave_flag[4];
+    __shared__ int wave_before[4];
     const long A = (long)g.batch * g.nodes;
     const long r0 = (long)blockIdx.x * rows_per;
     const int nrows = A - r0 < rows_per ? (int)(A - r0) : rows_per;
@@ -1060,75 +1130,21 @@ __global__ void __launch_bounds__(256) graph_fill_kernel(Grid g, Workspace w, in
         hit[k] = lane < cap ? (int)hits[r * cap + lane] : 0;     // (past the row's degree: not used)
         if (x) xi[k] = load3(x + 3 * r);
     }
-    if (blockIdx.x == 0) {                                        // the statistics of the whole graph: the host waits for them
-        long long all = 0;
-        int mx = 0, cell = 0, flag = 0;
-        const long n = tiled ? A / kScanTile + 1 : A;             // ceil((A + 1) / kScanTile) tiles
-        const int* sums = tiled ? w.deg_sums : w.degree;
-        const int* maxima = tiled ? w.deg_max : w.degree;
-        for (long k = tid; k < n; k += 256) {
-            all += sums[k];
-            const int m = maxima[k];
-            mx = m > mx ? m : mx;
-        }
-        for (int k = tid; k < n_box; k += 256) {
-            const int v = w.box_max[k] & ~kNanBit;
-            cell = v > cell ? v : cell;
-            flag |= w.box_max[k] & kNanBit;
-        }
-        for (int d = kWave / 2; d > 0; d >>= 1) {
-            all += __shfl_xor(all, d);
-            int t = __shfl_xor(mx, d);
-            mx = t > mx ? t : mx;
-            t = __shfl_xor(cell, d);
-            cell = t > cell ? t : cell;
-            flag |= __shfl_xor(flag, d);
-        }
-        if (lane == 0) {
-            wave_all[wave] = all;
-            wave_mx[wave] = mx;
-            wave_cell[wave] = cell;
-            wave_flag[wave] = flag;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            for (int k = 1; k < 4; k++) {
-                all += wave_all[k];
-                mx = wave_mx[k] > mx ? wave_mx[k] : mx;
-                cell = wave_cell[k] > cell ? wave_cell[k] : cell;
-                flag |= wave_flag[k];
-            }
-            // (a host may be polling these words: each is stored once, at system scope)
-            const int words[4] = {all > 0x7fffffffLL ? 0x7fffffff : (int)all, cell, mx,
-                                  (all > 0x7fffffffLL ? 1 : 0) | (flag ? 4 : 0)};
-#pragma unroll
-            for (int k = 0; k < 4; k++) __hip_atomic_store(stats + k, words[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
-    }
-    // of row r0 + lane
-    int my_degree, my_start;
+    if (blockIdx.x == 0) graph_statistics(w, A, tiled, n_box, stats);
+    FillRow own;                                                  // row r0 + lane
     if (tiled) {
-        // (scan_sums_kernel has left the sums inside the tile in the place of the degrees; a wave adds the tiles before by itself)
-        const int tile = (int)(r0 / kScanTile);
-        int incl = 0, prev = 0, before = 0;
-        if (lane < nrows) {
-            incl = w.degree[r0 + lane];
-            if ((r0 + lane) % kScanTile != 0) prev = w.degree[r0 + lane - 1];
-        }
-        for (int k = lane; k < tile; k += kWave) before += w.deg_sums[k];
-        for (int d = kWave / 2; d > 0; d >>= 1) before += __shfl_xor(before, d);
-        my_degree = incl - prev;
-        my_start = before + prev;
+        own = row_of_tile(w, r0, lane, nrows);
     } else {
-        my_degree = lane < nrows ? w.degree[r0 + lane] : 0;
+        own.degree = lane < nrows ? w.degree[r0 + lane] : 0;
         int before = 0;
         for (long r = tid; r < r0; r += 256) before += w.degree[r];
         for (int d = kWave / 2; d > 0; d >>= 1) before += __shfl_xor(before, d);
         if (lane == 0) wave_before[wave] = before;
-        const int incl = wave_incl_scan(my_degree, lane);         // (every wave by itself)
+        const int incl = wave_incl_scan(own.degree, lane);        // (every wave by itself)
         __syncthreads();
-        my_start = wave_before[0] + wave_before[1] + wave_before[2] + wave_before[3] + incl - my_degree;
+        own.start = wave_before[0] + wave_before[1] + wave_before[2] + wave_before[3] + incl - own.degree;
     }
+    const int my_degree = own.degree, my_start = own.start;
 
     const int my_box = (int)((unsigned)(r0 + (lane < nrows ? lane : 0)) / (unsigned)g.nodes) * g.nodes;      // first row of the row's box
     float3 xj[RW];
@@ -1160,19 +1176,86 @@ __global__ void __launch_bounds__(256) graph_fill_kernel(Grid g, Workspace w, in
             if (x) here.store_vector(t, wrapped_difference(load3(x + 3 * (long)j), xi[k], box));
         }
     }
-    if (wave == 0 && lane < nrows) {
-        row_ptr[r0 + lane] = my_start;
-        const long next = r0 + lane + 1;
-        if (next == A) row_ptr[A] = my_start + my_degree;
-        const unsigned q = (unsigned)next / (unsigned)g.nodes;                    // (next < 2^31: 32-bit divide)
-        if (q * (unsigned)g.nodes == (unsigned)next) edge_counts[q - 1] = my_start + my_degree;
-    }
+    if (wave == 0 && lane < nrows) put_row(g, A, r0 + lane, own, row_ptr, edge_counts);
     if (wave == 1 && lane < nrows && order) {
         const unsigned k = (unsigned)(r0 + lane);
         order[k] = (int)(k / (unsigned)g.nodes) * g.nodes + __float_as_int(w.sorted[k].w);
     }
 }
 
+// The same with the edges of 64 rows dealt out to the threads, which find their rows by bisection: for rows much shorter than a wave.
+constexpr int kFillUnroll = 4;
+template <typename HitT>
+__global__ void __launch_bounds__(256) graph_fill_dealt_kernel(Grid g, Workspace w, int n_box, int* __restrict__ row_ptr,
+                                                               int* __restrict__ edge_counts, int* stats, int capacity, EdgeOut out,
+                                                               int* __restrict__ order) {
+    constexpr int rows_per = kFillRows;
+    __shared__ int rp[kFillRows + 1];
+    __shared__ int first_row[kFillRows];      // first row of the box that the row belongs to
+    __shared__ float3 x_row[kFillRows];
+    const long A = (long)g.batch * g.nodes;
+    const long r0 = (long)blockIdx.x * rows_per;
+    const int nrows = A - r0 < rows_per ? (int)(A - r0) : rows_per;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    if (blockIdx.x == 0) graph_statistics(w, A, 1, n_box, stats);
+    if (wave == 0) {
+        const FillRow own = row_of_tile(w, r0, lane, nrows);
+        if (lane < nrows) {
+            rp[lane + 1] = own.start + own.degree;
+            put_row(g, A, r0 + lane, own, row_ptr, edge_counts);
+        }
+        if (lane == 0) rp[0] = own.start;
+        if (lane >= nrows && lane < rows_per) rp[lane + 1] = 0x7fffffff;
+    }
+    if (wave == 1 && lane < nrows) {
+        const unsigned k = (unsigned)(r0 + lane);
+        const int first = (int)(k / (unsigned)g.nodes) * g.nodes;
+        first_row[lane] = first;
+        if (order) order[k] = first + __float_as_int(w.sorted[k].w);
+    }
+    if (wave == 2 && lane < nrows && out.r_ij) x_row[lane] = load3(out.x + 3 * (r0 + lane));
+    __syncthreads();
+    const int cap = w.hit_cap;
+    const HitT* __restrict__ hits = static_cast<const HitT*>(w.hits);
+    const int e_hi = rp[nrows];
+    const Box3 box = box_of(g.bx, g.by, g.bz);
+    for (int e0 = rp[0] + tid; e0 < e_hi; e0 += 256 * kFillUnroll) {
+        int row[kFillUnroll], j[kFillUnroll];
+        bool ok[kFillUnroll];
+#pragma unroll
+        for (int u = 0; u < kFillUnroll; u++) {
+            const int e = e0 + 256 * u;
+            int lo = 0;                                // last row with rp <= e (rp ends in INT_MAX past the last row)
+            for (int step = rows_per >> 1; step > 0; step >>= 1) lo += rp[lo + step] <= e ? step : 0;
+            lo = lo < nrows ? lo : nrows - 1;          // (a position past the last edge: discarded below, but it must not
+                                                       // name a row that is not staged, its atom is read all the same)
+            const int idx = e - rp[lo], deg = rp[lo + 1] - rp[lo];
+            ok[u] = e < e_hi && deg <= cap && idx >= 0 && idx < deg && e >= 0 && e < capacity;
+            row[u] = lo;
+            j[u] = ok[u] ? (int)hits[(r0 + lo) * cap + idx] : 0;
+        }
+        float3 xj[kFillUnroll];
+#pragma unroll
+        for (int u = 0; u < kFillUnroll; u++) {
+            j[u] += first_row[row[u]];
+            if (out.r_ij) xj[u] = load3(out.x + 3 * (long)j[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kFillUnroll; u++)
+            if (ok[u]) out.store(e0 + 256 * u, (int)r0 + row[u], j[u]);
+        if (out.r_ij) {
+#pragma unroll
+            for (int u = 0; u < kFillUnroll; u++) {
+                const float3 r = wrapped_difference(xj[u], x_row[row[u]], box);
+                if (ok[u]) out.store_vector(e0 + 256 * u, r);
+            }
+        }
+    }
+    for (int r = wave; r < nrows; r += 4)
+        if (rp[r + 1] - rp[r] > cap) refill_row(g, w, (int)(r0 + r), rp[r], capacity, out);
+}
+
+// order[k] = global id of the k-th atom in cell order (cells x-major, atoms by id inside a cell)
 __global__ void __launch_bounds__(256) cell_order_kernel(Grid g, Workspace w, int* __restrict__ order) {
     const long A = (long)g.batch * g.nodes;
     const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1515,9 +1598,16 @@ int mg_graph_fill(const float* x, const void* workspace, size_t workspace_bytes,
         hipLaunchKernelGGL((graph_fill_kernel<decltype(hit), decltype(rw)::value>), dim3((unsigned)ceil_div(A, 4 * decltype(rw)::value)),
                            dim3(256), 0, st, g, w, tiled, box_max_entries(g), row_ptr, edge_counts, stats, capacity, out, order);
     };
+    // Rows that fill less than half of a wave's lanes are dealt out (131 072 rows of 26 edges: a whole search 101 us so, 103 with a wave to
+    // a row, 108 with half a wave to a row; of 52 edges 160, 146, 150)
+    const double mean = 4.18879 * cutoff * cutoff * cutoff * nodes / ((double)box_x * box_y * box_z);
+    const bool dealt = tiled && mean <= 32;
     auto with_rows = [&](auto hit) {
         if (A <= 4096) launch(hit, std::integral_constant<int, 1>{});
-        else launch(hit, std::integral_constant<int, 8>{});
+        else if (!dealt) launch(hit, std::integral_constant<int, 8>{});
+        else
+            hipLaunchKernelGGL(graph_fill_dealt_kernel<decltype(hit)>, dim3((unsigned)ceil_div(A, kFillRows)), dim3(256), 0, st, g, w,
+                               box_max_entries(g), row_ptr, edge_counts, stats, capacity, out, order);
     };
     if (w.hit_bytes == 2) with_rows((unsigned short)0);
     else with_rows((int)0);

@@ -393,3 +393,26 @@ def test_arrays_of_a_graph_are_little_longer_than_its_edges(pkg):
             if first is not None:
                 assert torch.equal(first[0], graph.dst) and torch.equal(first[1], r)
             first = graph.dst, r
+
+
+@pytest.mark.parametrize("batch,atoms,cutoff,side,clump", [
+    (3, 5501, 4.0, 38.3, 0), (1, 16385, 4.0, 55.0, 500),       # rows shorter than half a wave: edges dealt out; some longer than a hit row
+    (2, 8200, 5.0, 43.7, 0), (1, 17411, 6.0, 56.2, 400),       # a wave to a row, rows in several strides; a last tile of few rows
+    (1, 4097, 5.0, 34.7, 0), (5, 819, 5.0, 20.3, 300)])        # eight rows and one row to a wave without the scan of tiles
+def test_fill_pass_by_rows_and_by_edges(pkg, batch, atoms, cutoff, side, clump):
+    """Every branch of the fill pass against the two-call search (scan and fill kernels of their own): row pointer, edges in both widths,
+    vectors recomputed from them."""
+    ops = importlib.import_module("learned-dynamics_amd.ops")
+    gen = torch.Generator().manual_seed(atoms)
+    pos = torch.rand(batch, atoms, 3, generator=gen) * side
+    if clump:
+        pos[:, :clump] = 0.5 * side + 2 * torch.randn(batch, clump, 3, generator=gen)
+    pos = pos.cuda()
+    ext = importlib.import_module("learned-dynamics_amd._lib").load_torch_ext()
+    src32, dst32, src, dst, counts, row_ptr, order, r_ij = ext.radius_graph(256, 100000, cutoff, side, side, side, pos, True)
+    search = ops.NeighbourSearch(pos, cutoff, (side,) * 3)
+    want_src, want_dst = search.fill()
+    assert torch.equal(src32, want_src) and torch.equal(dst32, want_dst)
+    assert torch.equal(src, want_src.long()) and torch.equal(dst, want_dst.long())
+    assert torch.equal(row_ptr, search.row_ptr) and torch.equal(counts, search.edge_counts)
+    assert torch.equal(r_ij, ops.edge_vectors(pos.reshape(-1, 3), want_src, want_dst, (side,) * 3))
