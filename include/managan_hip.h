@@ -400,6 +400,14 @@ typedef struct mg_mlp_f16x2_grad {
 int mg_mlp_f16x2_supported(int dim_in, int dim);      /* returns 0 / 1, not a status */
 int mg_mlp_f16x2_forward(const mg_mlp_f16x2* args /* host */, mg_stream_t stream);
 int mg_mlp_f16x2_adjoint(const mg_mlp_f16x2_grad* args /* host */, mg_stream_t stream);
+/* The nonlinear layers of an MLP whose result is only needed summed over the rows of segments (archs/diffuser_atoms15.py:98-110
+ * under edges_reduce_src, :244-246): out[s] = sum over the rows r of segment s of f(W2 f(W1 x[r] + b1) + b2), f = LeakyReLU(0.1),
+ * x (rows, dim_in), both layers `dim` wide, out (n_out, dim).  Rows are sorted by segment (seg ascending, row_ptr its CSR form);
+ * sizes as mg_mlp_f16x2_supported.  workspace: 16-byte aligned.  Sums run in row order within blocks of 32 rows, then in block order. */
+int mg_mlp_leaky_rowsum_f16x2_workspace_bytes(long rows, int dim, size_t* bytes /* host */);
+int mg_mlp_leaky_rowsum_f16x2(const void* packed_W1, const float* b1, const void* packed_W2, const float* b2, const float* x,
+                              long rows, int dim_in, int dim, const int* row_ptr, const int* seg, long n_out, void* workspace,
+                              float* out, mg_stream_t stream);
 /* y = act(x W^T + bias) in float64 arithmetic: W (dim_out, dim_in) and bias are the float32 parameters, widened
  * exactly; x (rows, dim_in), every product and sum, the activation and y (rows, dim_out) are double.  The same
  * contraction as nn.Linear inside the reference's MLPs (archs/meanflow_painn8.py:38-51); float64 has no counterpart

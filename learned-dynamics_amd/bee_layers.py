@@ -247,8 +247,8 @@ class MLP(nn.Module):
         (n_out, d).  Only the first two layers are nonlinear: the direct linear and the last layer commute
         with the sum, so they run on the n_out summed rows instead of on every row:
             sum_e mlp(x_e) = (W_direct [+ I]) sum_e x_e + W_last sum_e h_e + (rows in the segment) b_last
-        with h = act(W_2 act(W_1 x + b_1) + b_2).  seg (rows,) int32: the segment of every row; with it the
-        second layer sums its output rows in its own epilogue and h is never stored.  s_x: sum_e x_e if the
+        with h = act(W_2 act(W_1 x + b_1) + b_2).  seg (rows,) int32: the segment of every row; with it both layers and the
+        sum are one kernel up to 512 columns, and the second layer sums its output rows in its own epilogue beyond.  s_x: sum_e x_e if the
         caller already has it; count (n_out, 1) float32: the rows per segment, if the caller has them.
         The scale is carried by the two node-level matrices and the bias (scaled copies cached with the weights).
         add_to (n_out, d) contiguous: the result is added to it in place (and it is returned)."""
@@ -259,17 +259,20 @@ class MLP(nn.Module):
         W_last = W_last0 if scale == 1.0 else _derived(self, ("last_scaled", scale), (W_last0,), lambda: scale * W_last0)
         b_last = b_last0 if scale == 1.0 else _derived(self, ("last_bias_scaled", scale), (b_last0,), lambda: scale * b_last0)
         L = self.layers
-        if bound is None and ops.get_linear_mode() == ops.LINEAR_F16X2:
-            bound = ops.row_absmax(x)
-        h, b1 = _linear(x, L[0].weight, L[0].bias, ops.ACT_LEAKY, bound)
-        if (seg is not None and b1 is not None
-                and ops.f16x2_rowsum_supported(h.shape[0], L[2].in_features, L[2].out_features, h)):
-            s_h, _ = ops.tensor_linear_f16x2_rowsum(L[2].weight, h, b1, row_ptr, seg, n_out, bias=L[2].bias,
-                                                    act=ops.ACT_LEAKY)
+        if seg is not None and ops.mlp_rowsum_supported(x.shape[0], L[0].in_features, L[0].out_features, x):
+            s_h = ops.mlp_leaky_rowsum(L[0].weight, L[0].bias, L[2].weight, L[2].bias, x, row_ptr, seg, n_out)
         else:
-            h, _ = _linear(h, L[2].weight, L[2].bias, ops.ACT_LEAKY, b1, want_bound=False)
-            s_h = ops.segment_sum_csr(h, row_ptr, n_out)
-        del h
+            if bound is None and ops.get_linear_mode() == ops.LINEAR_F16X2:
+                bound = ops.row_absmax(x)
+            h, b1 = _linear(x, L[0].weight, L[0].bias, ops.ACT_LEAKY, bound)
+            if (seg is not None and b1 is not None
+                    and ops.f16x2_rowsum_supported(h.shape[0], L[2].in_features, L[2].out_features, h)):
+                s_h, _ = ops.tensor_linear_f16x2_rowsum(L[2].weight, h, b1, row_ptr, seg, n_out, bias=L[2].bias,
+                                                        act=ops.ACT_LEAKY)
+            else:
+                h, _ = _linear(h, L[2].weight, L[2].bias, ops.ACT_LEAKY, b1, want_bound=False)
+                s_h = ops.segment_sum_csr(h, row_ptr, n_out)
+            del h
         if s_x is None:
             s_x = ops.segment_sum_csr(x, row_ptr, n_out)
         if add_to is None:

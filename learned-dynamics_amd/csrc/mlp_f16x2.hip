@@ -18,6 +18,7 @@
 // everywhere (78 us, 40 us): fewer waves to wait beside.
 #include "common.hpp"
 #include "f16x2.hpp"
+#include "rowsum_finish.hpp"
 #include "silu.hpp"
 
 namespace mg {
@@ -50,7 +51,8 @@ __device__ __forceinline__ bool has_marks(const float* inv, int O, int lane) {
 // acc[mi][ni] = rows (pieces in LDS, xh at the first row block, mi_stride halves between them, lo pieces x_lo halves further on)
 // times the 32 NI weight rows whose fragments start at wp.  The two small products of a step have an accumulator of their own, and
 // with SUMS = 2 the large ones have two: the large sum is rounded once per 16 or 32 k instead of three times per 16.
-template <int MI, int NI, int SUMS>
+// ROWS_FIRST: the rows are the A operand, and a lane holds sixteen rows of one column.
+template <int MI, int NI, int SUMS, bool ROWS_FIRST = false>
 __device__ __forceinline__ void multiply(const _Float16* __restrict__ wp, long w_lo, int K, const _Float16* xh, int mi_stride,
                                          int x_lo, int lane, floatx16 (&acc)[MI][NI]) {
     constexpr int kX = SUMS;                                       // (buffers of x: what the registers hold)
@@ -70,6 +72,9 @@ __device__ __forceinline__ void multiply(const _Float16* __restrict__ wp, long w
 #pragma unroll
                 for (int k = 0; k < SUMS; k++) large[k][mi][ni][q] = 0.f;
             }
+    auto mfma = [](const halfx8& w, const halfx8& x, const floatx16& c) {
+        return ROWS_FIRST ? __builtin_amdgcn_mfma_f32_32x32x16_f16(x, w, c, 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x16_f16(w, x, c, 0, 0, 0);
+    };
     auto load_w = [&](int u, int s) {
         const _Float16* p = wp + 512L * (s < steps ? s : steps - 1);      // (surplus loads of the last trip are never used)
 #pragma unroll
@@ -99,14 +104,14 @@ __device__ __forceinline__ void multiply(const _Float16* __restrict__ wp, long w
             for (int mi = 0; mi < MI; mi++)
 #pragma unroll
                 for (int ni = 0; ni < NI; ni++) {
-                    small[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wh[u][ni], bl[x][mi], small[mi][ni], 0, 0, 0);
-                    large[u % SUMS][mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wh[u][ni], bh[x][mi], large[u % SUMS][mi][ni], 0, 0, 0);
+                    small[mi][ni] = mfma(wh[u][ni], bl[x][mi], small[mi][ni]);
+                    large[u % SUMS][mi][ni] = mfma(wh[u][ni], bh[x][mi], large[u % SUMS][mi][ni]);
                 }
 #pragma unroll
             for (int mi = 0; mi < MI; mi++)
 #pragma unroll
                 for (int ni = 0; ni < NI; ni++)
-                    small[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wl[u][ni], bh[x][mi], small[mi][ni], 0, 0, 0);
+                    small[mi][ni] = mfma(wl[u][ni], bh[x][mi], small[mi][ni]);
             __builtin_amdgcn_sched_barrier(0);
             load_w(u, s + u + 2);
         }
@@ -173,6 +178,44 @@ __device__ __forceinline__ void swap_rows(float& a, float& b) {
     b = __uint_as_float(r[1]);
 }
 
+// The rows of x, row(mi, mm) in memory, as pieces, their maxima to row_max: eight lanes to a row, whole rows in registers
+// between the maximum and the split
+template <int MI, typename Row>
+__device__ __forceinline__ void split_rows(_Float16* xh, float* row_max, int K, bool marked, int wave, int waves, int lane, Row row_of) {
+    const int x_lo = 32 * MI * K, p = lane & 7;
+    for (int grp = wave; grp < 4 * MI; grp += waves) {
+        const int lr = grp * 8 + (lane >> 3), mi = lr >> 5, mm = lr & 31;
+        const float* row = row_of(mi, mm) + 4 * p;
+        float v[kMaxDim / 32][4];
+        float mx = 0.f;
+#pragma unroll
+        for (int j = 0; j < kMaxDim / 32; j++)
+            if (32 * j < K) {
+                const float4 f = *reinterpret_cast<const float4*>(row + 32 * j);
+                v[j][0] = f.x; v[j][1] = f.y; v[j][2] = f.z; v[j][3] = f.w;
+            }
+#pragma unroll
+        for (int j = 0; j < kMaxDim / 32; j++)
+            if (32 * j < K)
+#pragma unroll
+                for (int i = 0; i < 4; i++) mx = fmaxf(mx, fabsf(v[j][i]));
+#pragma unroll
+        for (int d = 1; d < 8; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
+        float inv;
+        const float scale = pow2_scale(mx, &inv);
+        const bool bits = marked || beyond_split(mx);
+        const int at = mi * 32 * K + piece_at(mm, 4 * p);
+#pragma unroll
+        for (int j = 0; j < kMaxDim / 32; j++)
+            if (32 * j < K) store_pieces(xh, x_lo, at + 1024 * j, v[j], scale);
+        if (__any(bits))                                           // (rare)
+#pragma unroll
+            for (int j = 0; j < kMaxDim / 32; j++)
+                if (32 * j < K && bits) store_bits(xh, x_lo, at + 1024 * j, v[j]);
+        if (p == 0) row_max[lr] = mx;
+    }
+}
+
 // DUAL: the 32 rows of a block are 16 values and their 16 tangents
 template <int MI, int NI, int MODE, bool DUAL>
 __global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const MlpArgs a) {
@@ -198,40 +241,9 @@ __global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const
 
     float isx[MI];
     bool odd[MI];
-    {   // the rows of x: eight lanes to a row, whole rows in registers between the maximum and the split
-        const int K = a.K, x_lo = TM * K, p = lane & 7;
+    {
         const bool marked = has_marks(a.inv[0], a.O, lane);
-        for (int grp = wave; grp < 4 * MI; grp += waves) {
-            const int lr = grp * 8 + (lane >> 3), mi = lr >> 5, mm = lr & 31;
-            const float* row = a.x + row_of(mi, mm) * K + 4 * p;
-            float v[kMaxDim / 32][4];
-            float mx = 0.f;
-#pragma unroll
-            for (int j = 0; j < kMaxDim / 32; j++)
-                if (32 * j < K) {
-                    const float4 f = *reinterpret_cast<const float4*>(row + 32 * j);
-                    v[j][0] = f.x; v[j][1] = f.y; v[j][2] = f.z; v[j][3] = f.w;
-                }
-#pragma unroll
-            for (int j = 0; j < kMaxDim / 32; j++)
-                if (32 * j < K)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) mx = fmaxf(mx, fabsf(v[j][i]));
-#pragma unroll
-            for (int d = 1; d < 8; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
-            float inv;
-            const float scale = pow2_scale(mx, &inv);
-            const bool bits = marked || beyond_split(mx);
-            const int at = mi * 32 * K + piece_at(mm, 4 * p);
-#pragma unroll
-            for (int j = 0; j < kMaxDim / 32; j++)
-                if (32 * j < K) store_pieces(xh, x_lo, at + 1024 * j, v[j], scale);
-            if (__any(bits))                                       // (rare)
-#pragma unroll
-                for (int j = 0; j < kMaxDim / 32; j++)
-                    if (32 * j < K && bits) store_bits(xh, x_lo, at + 1024 * j, v[j]);
-            if (p == 0) row_max[lr] = mx;
-        }
+        split_rows<MI>(xh, row_max, a.K, marked, wave, waves, lane, [&](int mi, int mm) { return a.x + row_of(mi, mm) * a.K; });
         __syncthreads();
 #pragma unroll
         for (int mi = 0; mi < MI; mi++) {
@@ -441,6 +453,179 @@ __global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const
     }
 }
 
+// Linear, LeakyReLU(0.1), Linear, LeakyReLU(0.1), then the sum over the rows of each segment (seg ascending); the hidden rows stay in
+// LDS and the second layer's in registers.  64 rows a workgroup, wave w owns 32 columns of both layers.  In the second
+// layer the rows are the A operand: a lane holds rows of ONE column, and after a swap of the halves of the wave lanes 0 .. 31
+// hold all rows of the first block of 32 and lanes 32 .. 63 those of the second, so that a segment's rows add up in row
+// order in a register, at 64 additions a wave.  Partial rows of segments that leave a block go to slots A / B (rowsum_finish.hpp).
+// A plain linear that stores its rows and a second that reads them and sums (the route for wider layers) took, with 256 -> 512 ->
+// 512 and 15 rows a segment, 446 us for 131 072 rows against 341 here, 109 and 98 for 32 768, 55 and 39 for 8192; 128 -> 256 149
+// and 106, 51 and 29, 38 and 18; 64 -> 128 80 and 42, 38 and 17, 22 and 16.  Bound as the kernel above: 0.9 PFLOP/s, counting the
+// three products, in long runs.
+struct RowsumArgs {
+    const float* x;
+    long R;
+    int K, O;
+    const _Float16* planes[2];
+    const float* inv[2];
+    const float* bias[2];
+    const int* seg;
+    long n_blocks;
+    float *slots, *out;
+};
+
+__device__ __forceinline__ float leaky(float v) { return v >= 0.f ? v : 0.1f * v; }
+
+__global__ void __launch_bounds__(64 * kMaxWaves, 4) mlp_rowsum_f16x2_kernel(const RowsumArgs a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    constexpr int MI = 2, TM = 32 * MI;
+    const int O = a.O, widest = a.K > O ? a.K : O;
+    _Float16* const xh = reinterpret_cast<_Float16*>(lds);
+    float* const row_max = reinterpret_cast<float*>(lds + (size_t)TM * widest * 4);      // [waves][TM]
+    float* const row_inv = row_max + kMaxWaves * TM;                                     // [TM]
+    float* const fixed = row_inv + TM;                                                   // [kMaxDim]
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
+    const int m = lane & 31, G = lane >> 5;
+    const long r0 = (long)blockIdx.x * TM;
+    // rows past the end repeat the last one and are not summed
+    auto row_of = [&](int r) { return r0 + r < a.R ? r0 + r : a.R - 1; };
+
+    float isx[MI];
+    bool odd[MI];
+    floatx16 acc[MI][1];
+    auto each_odd_row = [&](int l, int K, auto set) {              // set(mi, row, its sums in `fixed`)
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++) {
+            unsigned rows = (unsigned)__ballot(odd[mi]);
+            while (rows) {
+                const int r = __builtin_ctz(rows);
+                rows &= rows - 1;
+                for (int n = tid; n < O; n += blockDim.x)
+                    fixed[n] = lds_row_in_fp32(xh + mi * 32 * K, TM * K, r, a.planes[l], (long)pad256(O) * K, n, K, a.inv[l][n]);
+                __syncthreads();
+                set(mi, r);
+                __syncthreads();
+            }
+        }
+    };
+
+    {
+        const bool marked = has_marks(a.inv[0], O, lane);
+        split_rows<MI>(xh, row_max, a.K, marked, wave, waves, lane, [&](int mi, int mm) { return a.x + row_of(32 * mi + mm) * a.K; });
+        __syncthreads();
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++) {
+            const float mx = row_max[32 * mi + m];
+            pow2_scale(mx, &isx[mi]);
+            odd[mi] = marked || beyond_split(mx);
+        }
+        __syncthreads();                                           // (row_max is written again below)
+    }
+    multiply<MI, 1, 1>(a.planes[0] + (long)wave * (a.K >> 5) * 1024, (long)pad256(O) * a.K, a.K, xh, 32 * a.K, TM * a.K, lane, acc);
+    if (__any(odd[0] || odd[1]))
+        each_odd_row(0, a.K, [&](int mi, int r) {
+#pragma unroll
+            for (int q = 0; q < 16; q++) {
+                const float f = fixed[32 * wave + 8 * (q / 4) + 4 * G + q % 4];
+                if (m == r) acc[mi][0][q] = f;
+            }
+        });
+    float mx[MI] = {0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int col = 32 * wave + 8 * t + 4 * G;
+        const float4 w4 = *reinterpret_cast<const float4*>(a.inv[0] + col);
+        const float4 b4 = a.bias[0] ? *reinterpret_cast<const float4*>(a.bias[0] + col) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float iw[4] = {w4.x, w4.y, w4.z, w4.w}, b[4] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float p = acc[mi][0][4 * t + i];
+                const float v = leaky((odd[mi] ? p : p * isx[mi] * iw[i]) + b[i]);
+                acc[mi][0][4 * t + i] = v;
+                mx[mi] = fmaxf(mx[mi], fabsf(v));
+            }
+    }
+    const bool marked = has_marks(a.inv[1], O, lane);
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++) {
+        mx[mi] = fmaxf(mx[mi], __shfl_xor(mx[mi], 32));
+        if (G == 0) row_max[wave * TM + 32 * mi + m] = mx[mi];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++) {
+        float top = 0.f;
+        for (int w = 0; w < waves; w++) top = fmaxf(top, row_max[w * TM + 32 * mi + m]);
+        const float scale = pow2_scale(top, &isx[mi]);
+        odd[mi] = marked || beyond_split(top);
+        if (wave == 0 && G == 0) row_inv[32 * mi + m] = isx[mi];
+        auto each = [&](auto store) {
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const float v[4] = {acc[mi][0][4 * t], acc[mi][0][4 * t + 1], acc[mi][0][4 * t + 2], acc[mi][0][4 * t + 3]};
+                store(mi * 32 * O + piece_at(m, 32 * wave + 8 * t + 4 * G), v);
+            }
+        };
+        each([&](int at, const float (&v)[4]) { store_pieces(xh, TM * O, at, v, scale); });
+        if (__any(odd[mi]))                                        // (rare)
+            each([&](int at, const float (&v)[4]) { if (odd[mi]) store_bits(xh, TM * O, at, v); });
+    }
+    __syncthreads();
+
+    // second layer: lane = column 32 wave + m, register q = row 8 (q / 4) + 4 G + q % 4 of the block
+    multiply<MI, 1, 1, true>(a.planes[1] + (long)wave * (O >> 5) * 1024, (long)pad256(O) * O, O, xh, 32 * O, TM * O, lane, acc);
+    const int col = 32 * wave + m;
+    const float iw = a.inv[1][col], b = a.bias[1] ? a.bias[1][col] : 0.f;
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const float4 f = *reinterpret_cast<const float4*>(row_inv + 32 * mi + 8 * t + 4 * G);
+            const float inv[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[mi][0][4 * t + i] = acc[mi][0][4 * t + i] * inv[i] * iw + b;
+        }
+    if (__any(odd[0] || odd[1]))
+        each_odd_row(1, O, [&](int mi, int r) {
+            const float f = fixed[col] + b;
+#pragma unroll
+            for (int q = 0; q < 16; q++)
+                if (8 * (q / 4) + 4 * G + q % 4 == r) acc[mi][0][q] = f;
+        });
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(leaky(acc[0][0][q])), __float_as_uint(leaky(acc[1][0][q])), false, false);
+        acc[0][0][q] = __uint_as_float(s[0]);                      // row 8 (q / 4) + q % 4 of block G
+        acc[1][0][q] = __uint_as_float(s[1]);                      // row 8 (q / 4) + 4 + q % 4
+    }
+    const long left = a.R - r0 - 32 * G, block = 2 * (long)blockIdx.x + G;
+    const int rows = left < 32 ? (int)left : 32;                   // of this half's block; none if <= 0
+    const int my_seg = a.seg[row_of(lane)], before = __shfl_up(my_seg, 1);
+    const unsigned long long starts = __ballot(m > 0 && my_seg != before);
+    float* const slot = a.slots + (block < a.n_blocks ? block : 0) * O + col;
+    float* to = slot;                                              // of a block's first run; later ones lie inside the block
+    float sum = 0.f;
+#pragma unroll
+    for (int r = 0; r < 32; r++) {
+        if (r > 0 && (starts >> r & 0x100000001ull)) {
+            const int s_lo = __builtin_amdgcn_readlane(my_seg, r), s_hi = __builtin_amdgcn_readlane(my_seg, 32 + r);
+            if (starts >> (r + 32 * G) & 1) {                      // (never at a row past the end)
+                *to = sum;
+                sum = 0.f;
+                to = a.out + (long)(G ? s_hi : s_lo) * O + col;
+            }
+        }
+        const float v = acc[r >> 2 & 1][0][4 * (r >> 3) + (r & 3)];
+        sum += r < rows ? v : 0.f;
+    }
+    if (rows <= 0) return;
+    if (to != slot && rows == 32) to = a.slots + (a.n_blocks + block) * O + col;
+    *to = sum;
+}
+
 template <int MI, int NI, int MODE, bool DUAL>
 int launch(const MlpArgs& a, hipStream_t st) {
     const auto kernel = mlp_f16x2_kernel<MI, NI, MODE, DUAL>;
@@ -546,6 +731,50 @@ int mg_mlp_f16x2_adjoint(const mg_mlp_f16x2_grad* p, mg_stream_t stream) {
     MG_REQUIRE(fill(a, packed, a.O, a.O, a.N) && packed[0] && packed[1] && (packed[2] || !a.y) && a.x && aligned16(a.x) && aligned16(a.y),
                "mg_mlp_f16x2_adjoint: null or unaligned pointer");
     return choose<kAdjoint>(a, p->dual, (hipStream_t)stream);
+}
+
+int mg_mlp_leaky_rowsum_f16x2_workspace_bytes(long rows, int dim, size_t* bytes) {
+    MG_REQUIRE(bytes != nullptr && rows >= 0 && dim >= 0, "mg_mlp_leaky_rowsum_f16x2_workspace_bytes: bad argument");
+    *bytes = (size_t)(2 * ceil_div(rows, 32) * dim) * sizeof(float);
+    return MG_OK;
+}
+
+int mg_mlp_leaky_rowsum_f16x2(const void* packed_W1, const float* b1, const void* packed_W2, const float* b2, const float* x,
+                              long rows, int dim_in, int dim, const int* row_ptr, const int* seg, long n_out, void* workspace,
+                              float* out, mg_stream_t stream) {
+    MG_REQUIRE(mg_mlp_f16x2_supported(dim_in, dim), "mg_mlp_leaky_rowsum_f16x2: dimensions must be multiples of 32 up to %d", kMaxDim);
+    MG_REQUIRE(rows >= 0 && n_out >= 0 && rows < (1L << 31) && n_out < (1L << 31), "mg_mlp_leaky_rowsum_f16x2: bad size");
+    if (n_out == 0) return MG_OK;
+    MG_REQUIRE(row_ptr && out && aligned16(out), "mg_mlp_leaky_rowsum_f16x2: null or unaligned output");
+    hipStream_t st = (hipStream_t)stream;
+    RowsumArgs a{};
+    a.x = x;
+    a.R = rows;
+    a.K = dim_in;
+    a.O = dim;
+    a.seg = seg;
+    a.n_blocks = ceil_div(rows, 32);
+    a.slots = static_cast<float*>(workspace);
+    a.out = out;
+    if (rows > 0) {
+        const void* packed[2] = {packed_W1, packed_W2};
+        const float* bias[2] = {b1, b2};
+        for (int l = 0; l < 2; l++) {
+            MG_REQUIRE(packed[l] && aligned16(packed[l]) && (!bias[l] || aligned16(bias[l])), "mg_mlp_leaky_rowsum_f16x2: null or unaligned weight or bias");
+            a.planes[l] = static_cast<const _Float16*>(packed[l]);
+            a.inv[l] = reinterpret_cast<const float*>(a.planes[l] + 2L * ((dim + 255) / 256 * 256) * (l == 0 ? dim_in : dim));
+            a.bias[l] = bias[l];
+        }
+        MG_REQUIRE(x && seg && workspace && aligned16(x) && aligned16(workspace), "mg_mlp_leaky_rowsum_f16x2: null or unaligned row operand");
+        const int widest = dim_in > dim ? dim_in : dim;
+        const size_t lds = (size_t)64 * widest * 4 + (kMaxWaves * 64 + 64 + kMaxDim) * sizeof(float);
+        if (lds > 65536)
+            MG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mlp_rowsum_f16x2_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(mlp_rowsum_f16x2_kernel, dim3((unsigned)ceil_div(rows, 64)), dim3(2 * dim), lds, st, a);
+        if (int code = check_launch("mg_mlp_leaky_rowsum_f16x2")) return code;
+    }
+    rowsum_finish_kernel<<<dim3((unsigned)ceil_div(n_out * (dim / 4), 256)), dim3(256), 0, st>>>(row_ptr, n_out, a.n_blocks, dim, a.slots, 1.f, out);
+    return check_launch("rowsum_finish_kernel");
 }
 
 }  // extern "C"

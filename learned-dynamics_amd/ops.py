@@ -1927,6 +1927,38 @@ def tensor_linear_f16x2_rowsum(W, x, x_bound, row_ptr, seg, n_out, bias=None, ac
     return out, y
 
 
+def mlp_rowsum_supported(rows, dim_in, dim, x):
+    """mlp_leaky_rowsum takes these sizes.  Below 4096 rows (64 workgroups) a linear that splits its reduction and a plain
+    segment sum stay; from there on the one kernel is faster at every size (4096 rows: 256 -> 512 38 against 52 us, 32 -> 64 17 and 20)."""
+    return (get_linear_mode() == LINEAR_F16X2 and rows >= 4096 and x.data_ptr() % 16 == 0
+            and bool(_lib.mg_mlp_f16x2_supported(int(dim_in), int(dim))))
+
+
+def mlp_leaky_rowsum(W1, b1, W2, b2, x, row_ptr, seg, n_out):
+    """out[s] = sum over the rows r of segment s of f(W2 f(W1 x[r] + b1) + b2) with f = LeakyReLU(0.1): (n_out, dim).  Rows are
+    sorted by segment: seg (rows,) int32 ascending, row_ptr its CSR form.  The hidden rows are never stored."""
+    for t, nm in ((W1, "W1"), (W2, "W2"), (x, "x"), (b1, "b1"), (b2, "b2")):
+        if t is not None or nm in ("W1", "W2", "x"):
+            _check_input(t, nm)
+    for t, nm in ((row_ptr, "row_ptr"), (seg, "seg")):
+        _check_input(t, nm, torch.int32)
+    rows, dim_in, dim = int(x.size(0)), int(W1.size(1)), int(W1.size(0))
+    if x.dim() != 2 or x.size(1) != dim_in or tuple(W2.shape) != (dim, dim):
+        raise RuntimeError("x must have shape (rows, dim_in), W1 (dim, dim_in) and W2 (dim, dim)")
+    if any(b is not None and b.numel() != dim for b in (b1, b2)):
+        raise RuntimeError("the biases must have dim elements")
+    if seg.numel() != rows or row_ptr.numel() != n_out + 1:
+        raise RuntimeError("seg must have one entry per row and row_ptr n_out + 1 entries")
+    nbytes = ctypes.c_size_t(0)
+    L.check(_lib.mg_mlp_leaky_rowsum_f16x2_workspace_bytes(rows, dim, ctypes.byref(nbytes)))
+    with _on(x.device):
+        out = torch.empty(n_out, dim, dtype=torch.float32, device=x.device)
+        work = torch.empty(nbytes.value // 4, dtype=torch.float32, device=x.device)
+        L.check(_lib.mg_mlp_leaky_rowsum_f16x2(_p(packed_weight_f16x2(W1)), _p(b1), _p(packed_weight_f16x2(W2)), _p(b2), _p(x),
+                                               rows, dim_in, dim, _p(row_ptr), _p(seg), int(n_out), _p(work), _p(out), _stream()))
+    return out
+
+
 def painn_filter_hidden_supported(n_rbf, hidden, n_edges):
     """First two filter layers in one kernel: 16 radial functions, hidden width 256 or 512."""
     return get_linear_mode() == LINEAR_F16X2 and n_rbf == 16 and hidden in (256, 512) and n_edges >= 1024

@@ -128,3 +128,51 @@ def test_mlp_adjoint_of_a_row_beyond_the_pieces(ops, rows, dim):
     assert torch.equal(g_x[same], clean[same])
     assert not bool(torch.isfinite(g_x[rows - 2]).any())
     assert float((g_x[5].double() * 2.0 ** -100 - clean[5].double()).norm() / clean[5].double().norm()) <= 1.5e-6
+
+
+def _segments(rows, seed):
+    """Segments that begin and end anywhere in the blocks of 32 rows: empty ones, ones of one row, of a block, of several."""
+    g = torch.Generator().manual_seed(seed)
+    deg = torch.tensor([0, 32, 1, 31, 0, 0, 33, 30, 1, 64, 200, 2, 29, 3, 95, 1])
+    deg = torch.cat([deg, torch.randint(0, 40, (rows // 10 + 8,), generator=g)])
+    ends = deg.cumsum(0).clamp(max=rows)
+    ends[-1] = rows
+    row_ptr = torch.cat([torch.zeros(1, dtype=torch.long), ends])
+    return row_ptr, torch.repeat_interleave(torch.arange(ends.numel()), row_ptr[1:] - row_ptr[:-1])
+
+
+def _layers_and_sum(x, W, b, seg, n_out):
+    f = torch.nn.functional
+    h = x
+    for k in range(2):
+        h = f.leaky_relu(h @ W[k].to(x.dtype).t() + b[k].to(x.dtype), 0.1)
+    zero = torch.zeros(n_out, h.shape[1], dtype=x.dtype, device=x.device)
+    return zero.index_add(0, seg, h), torch.zeros(n_out, dtype=x.dtype, device=x.device).index_add(0, seg, h.norm(dim=1))
+
+
+@pytest.mark.parametrize("rows, dim_in, dim", [(1, 64, 64), (33, 512, 32), (64, 96, 288), (700, 160, 512), (4161, 256, 512), (5000, 32, 96)])
+def test_mlp_summed_over_segments(ops, rows, dim_in, dim):
+    """Against the formula in float64, relative to the sum of the segment's row norms: two layers of rows as above and sums of
+    up to 200 rows of which each addition rounds by 6e-8."""
+    W, b = (t[:2] for t in _weights(dim_in, dim))
+    g = torch.Generator().manual_seed(rows)
+    x = (torch.randn(rows, dim_in, generator=g) * torch.exp(2 * torch.randn(rows, 1, generator=g))).cuda()
+    row_ptr, seg = (t.cuda() for t in _segments(rows, rows))
+    n_out = row_ptr.numel() - 1
+    args = (row_ptr.int(), seg.int(), n_out)
+    out = ops.mlp_leaky_rowsum(W[0], b[0], W[1], b[1], x, *args)
+    ref, size = _layers_and_sum(x.double(), W, b, seg, n_out)
+    assert float(((out.double() - ref).norm(dim=1) / size.clamp_min(1e-30)).max()) <= 1.5e-6
+    assert not bool(out[row_ptr[1:] == row_ptr[:-1]].any())
+    assert torch.equal(ops.mlp_leaky_rowsum(W[0], b[0], W[1], b[1], x, *args), out)
+    # rows and a weight that the pieces cannot carry stay in their segments
+    x[rows // 2] *= 2.0 ** 110
+    x[0, 1] = INF
+    odd = ops.mlp_leaky_rowsum(W[0], b[0], W[1], b[1], x, *args)
+    hit = torch.zeros(n_out, dtype=torch.bool, device="cuda")
+    hit[seg[[0, rows // 2]]] = True
+    assert torch.equal(odd[~hit], out[~hit]) and not bool(torch.isfinite(odd[seg[0]]).any())
+    if int(seg[rows // 2]) != int(seg[0]):
+        big, size = _layers_and_sum(x.double(), W, b, seg, n_out)
+        k = seg[rows // 2]
+        assert float((odd[k].double() - big[k]).norm() / size[k]) <= 1.5e-6
