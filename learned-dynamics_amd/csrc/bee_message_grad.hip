@@ -13,7 +13,8 @@
 // node and not twice per edge; no filters are formed in memory.  dl leaves component-major (E, 13, chan), whole 256-byte
 // rows, and a second kernel sums it over the edges of each destination in a fixed order.
 // What bounds it: traffic, 17 floats read and 14 written per edge and channel, then 13 read.  131 000 edges, 8192 nodes, 256
-// channels, edge vectors not differentiated: 0.72 ms (5.8 TB/s) and 0.42 ms (4.2 TB/s).  Before, the filters were stored
+// channels, edge vectors not differentiated: 0.70 ms (6.0 TB/s) and 0.44 ms (4.1 TB/s).  Operands and gradients are component-major,
+// a wave's accesses 256 bytes each: the results of the forward kernel and of the output linears as they are.  Before, the filters were stored
 // (0.44 ms), two kernels gathered the 60 gradients at every edge's source (1.8 ms each), a third took the right operands'
 // gradients to enc and rh (0.35 ms) and three segment sums followed (0.37 ms).
 // Any multiple of 64 channels; differentiable.message_products comes here for multiples of 256, the widths of its forward
@@ -36,24 +37,22 @@ __device__ __forceinline__ void cross3(const float* a, const float* b, float* o)
     o[1] = a[2] * b[0] - a[0] * b[2];
     o[2] = a[0] * b[1] - a[1] * b[0];
 }
+// T values `stride` apart
 template <int T>
-__device__ __forceinline__ void load(const float* p, long row, int C, int c, float* o) {
-    const float* q = p + (row * C + c) * T;
+__device__ __forceinline__ void load(const float* p, long stride, float* o) {
 #pragma unroll
-    for (int k = 0; k < T; k++) o[k] = q[k];
+    for (int k = 0; k < T; k++) o[k] = p[k * stride];
 }
 
 __device__ __forceinline__ EdgeIn load_edge(const mg_bee_message_grad& a, long e, int node, int c) {
     EdgeIn in;
-    load<1>(a.l_0, node, a.chan, c, in.l);
-    load<3>(a.l_1, node, a.chan, c, in.l + 1);
-    load<9>(a.l_2, node, a.chan, c, in.l + 4);
-    in.enc = a.enc[e * a.chan + c];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        in.s[k] = a.dy[k][e * a.chan + c];
-        in.u[k] = a.rh[3 * e + k];
-    }
+    const long C = a.chan;
+    in.l[0] = a.l_0[node * C + c];
+    load<3>(a.l_1 + node * 3 * C + c, C, in.l + 1);
+    load<9>(a.l_2 + node * 9 * C + c, C, in.l + 4);
+    in.enc = a.enc[e * C + c];
+    load<3>(a.d_P0 + e * 3 * C + c, C, in.s);
+    load<3>(a.rh + 3 * e, 1, in.u);
     return in;
 }
 
@@ -71,16 +70,18 @@ __global__ void __launch_bounds__(256, 3) bee_message_grad_kernel(mg_bee_message
     const long begin = a.row_ptr[node], end = a.row_ptr[node + 1];
     if (begin >= end) return;
     float g011[3], g101[3], g121[3], g211[3], g111[3], g022[9], g202[9], g112[9], g222[9], g212[9];
-    load<3>(a.dy[3], node, C, c, g011);
-    load<3>(a.dy[4], node, C, c, g101);
-    load<3>(a.dy[5], node, C, c, g121);
-    load<3>(a.dy[6], node, C, c, g211);
-    load<9>(a.dy[7], node, C, c, g022);
-    load<9>(a.dy[8], node, C, c, g202);
-    load<9>(a.dy[9], node, C, c, g112);
-    load<9>(a.dy[10], node, C, c, g222);
-    load<3>(a.dy[11], node, C, c, g111);
-    load<9>(a.dy[12], node, C, c, g212);
+    const float *s1 = a.d_S1 + (long)node * 15 * C + c, *s2 = a.d_S2 + (long)node * 45 * C + c;
+    const long step = 5L * C;
+    load<3>(s1, step, g011);
+    load<3>(s1 + C, step, g101);
+    load<3>(s1 + 2 * C, step, g121);
+    load<3>(s1 + 3 * C, step, g211);
+    load<3>(s1 + 4 * C, step, g111);
+    load<9>(s2, step, g022);
+    load<9>(s2 + C, step, g202);
+    load<9>(s2 + 2 * C, step, g112);
+    load<9>(s2 + 3 * C, step, g222);
+    load<9>(s2 + 4 * C, step, g212);
     auto destination = [&](long e) {
         const int d = a.dst[e];
         return d < 0 ? 0 : (d >= a.n_rows ? a.n_rows - 1 : d);
@@ -186,12 +187,11 @@ __global__ void __launch_bounds__(256) bee_message_grad_sum_kernel(const float* 
 #pragma unroll
         for (int j = 0; j < kLeft; j++) s[j] += p[(long)j * C];
     }
-    const long at = (long)node * C + c;
-    d_0[at] = s[0];
+    d_0[(long)node * C + c] = s[0];
 #pragma unroll
-    for (int j = 0; j < 3; j++) d_1[3 * at + j] = s[1 + j];
+    for (int j = 0; j < 3; j++) d_1[((long)node * 3 + j) * C + c] = s[1 + j];
 #pragma unroll
-    for (int j = 0; j < 9; j++) d_2[9 * at + j] = s[4 + j];
+    for (int j = 0; j < 9; j++) d_2[((long)node * 9 + j) * C + c] = s[4 + j];
 }
 
 // floats of the two pieces of the workspace: the operands' gradients per edge, and d_rh's sums per 64 channels
@@ -234,9 +234,8 @@ int mg_bee_message_grad_run(const mg_bee_message_grad* args, mg_stream_t stream)
     MG_REQUIRE(items < (1L << 31) - 64 && sums < (1L << 31) - 64, "mg_bee_message_grad_run: too many nodes");
     float *dl = static_cast<float*>(a.workspace), *part = dl + (left ? left_floats(a.E, a.chan) : 0);
     if (a.E > 0 && (left || right || vec)) {
-        MG_REQUIRE(a.row_ptr && a.dst && a.rh && a.enc && a.l_0 && a.l_1 && a.l_2 && a.n_rows > 0 && (a.workspace || !(left || vec)),
+        MG_REQUIRE(a.row_ptr && a.dst && a.rh && a.enc && a.l_0 && a.l_1 && a.l_2 && a.d_P0 && a.d_S1 && a.d_S2 && a.n_rows > 0 && (a.workspace || !(left || vec)),
                    "mg_bee_message_grad_run: null pointer");
-        for (int k = 0; k < 13; k++) MG_REQUIRE(a.dy[k], "mg_bee_message_grad_run: gradient %d is null", k);
         const long per_xcd = ceil_div(ceil_div(items, 4), kXcds);
         if (left && right) launch<true, true>(a, vec, items, per_xcd, dl, part, st);
         else if (left) launch<true, false>(a, vec, items, per_xcd, dl, part, st);

@@ -215,8 +215,10 @@ __device__ __forceinline__ void lds_barrier() {
 // (waves per SIMD that the registers of the narrow tiles are held to: the epilogue's rare paths would cost one otherwise)
 constexpr int streaming_waves(int waves, int ni) { return waves == 4 && ni <= 2 ? 6 - ni : 1; }
 
-template <int WAVES, int NI>
-__global__ void __launch_bounds__(64 * WAVES, streaming_waves(WAVES, NI))
+// APART: the two small products of a step have an accumulator of their own, so that the large sum is rounded once per 16 k and not
+// three times (apart_of)
+template <int WAVES, int NI, bool APART>
+__global__ void __launch_bounds__(64 * WAVES, APART ? 1 : streaming_waves(WAVES, NI))
 linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restrict__ w_inv, const float* __restrict__ X,
                          const float* __restrict__ xmax, int xmax_parts, long xmax_stride, long xmax_div, long R, int I,
                          int O, int O_pad, const float* __restrict__ bias, int act, int accumulate,
@@ -251,6 +253,10 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
     for (int ni = 0; ni < NI; ni++)
 #pragma unroll
         for (int q = 0; q < 16; q++) acc[ni][q] = 0.f;
+    floatx16 apart[APART ? NI : 1];
+    if constexpr (APART)
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++) apart[ni] = acc[ni];
 
     // this lane's row of x (clamped past the end: those accumulators are never written)
     const long my_row = r0 + wave * 32 + m;
@@ -315,8 +321,9 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
                 const halfx8 bh = *reinterpret_cast<const halfx8*>(buf + b_off + 2048 * ni + 1024 * s);
                 const halfx8 bl = *reinterpret_cast<const halfx8*>(buf + kPlaneW + b_off + 2048 * ni + 1024 * s);
                 // small terms first
-                acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[s], bh, acc[ni], 0, 0, 0);
-                acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s], bl, acc[ni], 0, 0, 0);
+                floatx16& small = APART ? apart[APART ? ni : 0] : acc[ni];
+                small = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[s], bh, small, 0, 0, 0);
+                small = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s], bl, small, 0, 0, 0);
                 acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s], bh, acc[ni], 0, 0, 0);
             }
         order_chunk<NI>();
@@ -357,6 +364,9 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
         load_a(a1, k0 + 3 * kCK);
         __syncthreads();
     }
+    if constexpr (APART)
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++) acc[ni] += apart[ni];
 
     if constexpr (kRuns)
         if (out_T == 9) {                                    // (epilogue_runs has barriers: all waves go the same way)
@@ -737,7 +747,18 @@ inline Shape choose_shape(long R, int I, int O) {
     return s;
 }
 
-template <int WAVES, int NI>
+// A reduction of more than 512 in tiles of at most 128 columns keeps the small products apart, in a second set of accumulators.
+// The five rank-1 or rank-2 products of the message layers side by side, K = 1280, against float64: 2.7e-7 of the
+// result's 2-norm; in one accumulator 4.3e-7, five linears of K = 256 and a sum 3.5e-7, in fp32 6.5e-7.  Sequential
+// reductions take such a tile for every width; others keep the 256-column tile, which has no registers for the second set.
+inline bool apart_of(int I, int ni) { return I > 512 && ni <= 4; }
+inline Shape choose_sequential(long R, int I, int O) {
+    Shape s = choose_shape(R, I, O);
+    if (I > 512 && s.ni == 8) s.ni = 4;
+    return s;
+}
+
+template <int WAVES, int NI, bool APART = false>
 int launch(const _Float16* planes, const float* w_inv, const float* x, const float* xmax, int parts, long stride,
            long div, long rows, int I, int O, int O_pad, const float* bias, int act, int accumulate, float* y,
            float* ymax, int out_T, float bound_mul, float bound_add, long bias_rows, hipStream_t st) {
@@ -746,7 +767,7 @@ int launch(const _Float16* planes, const float* w_inv, const float* x, const flo
     const long total = tiles_m * tiles_n;
     const long grid = ceil_div(total, 8) * 8;
     MG_REQUIRE(grid <= 0x7fffffffL, "mg_tensor_linear_f16x2: grid too large (rows=%ld dim_out=%d)", rows, O);
-    hipLaunchKernelGGL((linear_rows_f16x2_kernel<WAVES, NI>), dim3((unsigned)grid), dim3(64 * WAVES), 0, st, planes,
+    hipLaunchKernelGGL((linear_rows_f16x2_kernel<WAVES, NI, APART>), dim3((unsigned)grid), dim3(64 * WAVES), 0, st, planes,
                        w_inv, x, xmax, parts, stride, div, rows, I, O, O_pad, bias, act, accumulate, y, ymax, tiles_n,
                        total, out_T, bound_mul, bound_add, bias_rows);
     return check_launch("mg_tensor_linear_f16x2");
@@ -831,7 +852,7 @@ int mg_components_to_rows(const float* x, long rows, int dim, int comps, int dim
 }
 
 int mg_tensor_linear_f16x2_rowmax_parts_sequential(long rows, int dim_in, int dim_out) {
-    return (int)ceil_div(dim_out, 32 * choose_shape(rows, dim_in, dim_out).ni);
+    return (int)ceil_div(dim_out, 32 * choose_sequential(rows, dim_in, dim_out).ni);
 }
 
 int mg_tensor_linear_f16x2_rowmax_parts(long rows, int dim_in, int dim_out) {
@@ -904,14 +925,24 @@ int mg_tensor_linear_f16x2_run(const mg_f16x2_linear* args, mg_stream_t stream) 
 #undef MG_SPLITK
         return check_launch("mg_tensor_linear_f16x2");
     }
-    Shape sh = choose_shape(a.rows, a.dim_in, a.dim_out);
+    Shape sh = a.sequential ? choose_sequential(a.rows, a.dim_in, a.dim_out) : choose_shape(a.rows, a.dim_in, a.dim_out);
     // nine components and a short reduction: bound by the stores, in runs out of this tile (18 432 x 32 -> 256 17 against 19 us,
     // 73 728 rows 40 against 65); longer reductions keep the tile that re-reads x least
     if (a.out_comps == 9 && a.dim_in <= 64 && a.dim_out % 64 == 0 && a.act == 0 && a.bias == nullptr) sh = Shape{2, 4};
-#define MG_F16X2_LAUNCH(WV, N)                                                                                             \
-    return launch<WV, N>(planes, w_inv, a.x, a.x_rowmax, a.x_rowmax_parts, a.x_rowmax_stride, a.x_rows_per_bound, a.rows,  \
+#define MG_F16X2_LAUNCH(WV, ...)                                                                                           \
+    return launch<WV, __VA_ARGS__>(planes, w_inv, a.x, a.x_rowmax, a.x_rowmax_parts, a.x_rowmax_stride, a.x_rows_per_bound, a.rows, \
                          a.dim_in, a.dim_out, O_pad, a.bias, a.act, a.accumulate, a.y, a.y_rowmax, a.out_comps,            \
                          a.bound_mul, a.bound_add, a.bias_rows, st)
+    if (apart_of(a.dim_in, sh.ni)) {
+        if (sh.waves == 8) {
+            if (sh.ni == 1) MG_F16X2_LAUNCH(8, 1, true);
+            if (sh.ni == 2) MG_F16X2_LAUNCH(8, 2, true);
+            MG_F16X2_LAUNCH(8, 4, true);
+        }
+        if (sh.ni == 1) MG_F16X2_LAUNCH(4, 1, true);
+        if (sh.ni == 2) MG_F16X2_LAUNCH(4, 2, true);
+        MG_F16X2_LAUNCH(4, 4, true);
+    }
     if (sh.waves == 8) {
         if (sh.ni == 1) MG_F16X2_LAUNCH(8, 1);
         if (sh.ni == 2) MG_F16X2_LAUNCH(8, 2);

@@ -267,7 +267,10 @@ constexpr int kFRowW = 64;                         // bytes per LDS row: 32 halv
 constexpr int kFPlane = kFTile * kFRowW;           // bytes of one piece of one operand
 constexpr int kFBuf = 4 * kFPlane;                 // one stage: two operands x two pieces
 constexpr int kFParts = 1024;                      // partial maxima per operand
-constexpr int kFRun = 4096;                        // rows per accumulation run (a multiple of kFRows)
+// rows per accumulation run (a multiple of kFRows).  Slices get longer the more tiles a product has: 27 000 rows of 16 x 1280 are
+// 1080 a slice, whose weights' gradients were off by 4.8e-7 of their 2-norm in one run and are by 3.4e-7 in runs of 256 (as the
+// five products of 16 x 256, 211 rows a slice, were); the additions do not show in the time.
+constexpr int kFRun = 256;
 
 // parts[b] = max |x| over the b-th share of n floats (n % 4 == 0, x 16-byte aligned)
 __global__ void __launch_bounds__(256) absmax_parts_kernel(const float* __restrict__ x, long n,

@@ -1252,8 +1252,7 @@ std::tuple<Tensors, OptTensor, OptTensor> bee_message_bwd(const Tensors& left, c
                                                           const Tensors& dy, const at::Tensor& row_ptr, const at::Tensor& dst,
                                                           const at::Tensor& dst_row_ptr, const OptTensor& perm, bool want_left,
                                                           bool want_enc, bool want_rh) {
-    static const int rank_of[13] = {0, 0, 0, 1, 1, 1, 1, 2, 2, 2, 2, 1, 2};
-    TORCH_CHECK(left.size() == 3 && dy.size() == 13, "bee_message_bwd: three operands and 13 gradients expected");
+    TORCH_CHECK(left.size() == 3 && dy.size() == 3, "bee_message_bwd: three operands and three gradients expected");
     check_input(enc, "enc");
     check_input(rh, "rh");
     check_input(row_ptr, "row_ptr", at::kInt);
@@ -1262,7 +1261,7 @@ std::tuple<Tensors, OptTensor, OptTensor> bee_message_bwd(const Tensors& left, c
     if (perm.has_value()) check_input(*perm, "perm", at::kInt);
     TORCH_CHECK(enc.dim() == 2 && rh.dim() == 2, "bee_message_bwd: enc (edges, chan) and rh (edges, 3) expected");
     const int64_t E = enc.size(0), C = enc.size(1), rows = left[0].size(0), n_src = row_ptr.numel() - 1;
-    const int64_t per_rank[3] = {C, 3 * C, 9 * C};
+    const int64_t per_rank[3] = {C, 3 * C, 9 * C}, wanted[3] = {E * 3 * C, n_src * 15 * C, n_src * 45 * C};
     TORCH_CHECK(rh.numel() == 3 * E && dst.numel() == E && dst_row_ptr.numel() == rows + 1 && n_src >= 0 &&
                     (!perm.has_value() || perm->numel() == E),
                 "bee_message_bwd: operand sizes");
@@ -1270,12 +1269,12 @@ std::tuple<Tensors, OptTensor, OptTensor> bee_message_bwd(const Tensors& left, c
     for (int k = 0; k < 3; k++) {
         check_input(left[k], "left operand");
         TORCH_CHECK(left[k].numel() == rows * per_rank[k], "bee_message_bwd: operand sizes");
+        check_input(dy[k], "gradient of the products");
+        TORCH_CHECK(dy[k].numel() == wanted[k], "bee_message_bwd: gradient sizes");
     }
-    for (int k = 0; k < 13; k++) {
-        check_input(dy[k], "gradient of a product");
-        TORCH_CHECK(dy[k].numel() == (rank_of[k] ? n_src : E) * per_rank[rank_of[k]], "bee_message_bwd: gradient sizes");
-        a.dy[k] = fp(dy[k]);
-    }
+    a.d_P0 = fp(dy[0]);
+    a.d_S1 = fp(dy[1]);
+    a.d_S2 = fp(dy[2]);
     c10::hip::HIPGuardMasqueradingAsCUDA guard(enc.device());
     Tensors d_left;
     if (want_left)

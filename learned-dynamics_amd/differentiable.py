@@ -913,12 +913,28 @@ def _message_products_plain(a_node, v_node, d_node, enc, rh, by_dst, by_src):
     return tuple(p if lab[2] == "0" else gl._ScatterSum.apply(p.contiguous(), by_src) for lab, p in zip(BEE_ORDER, prods))
 
 
-_S1_LABELS, _S2_LABELS = ("011", "101", "121", "211", "111"), ("022", "202", "112", "222", "212")
+def _by_component(*tensors):
+    """(rows, chan, 3, ..) as (rows, 3^rank, chan)"""
+    return tuple(t.flatten(2).transpose(1, 2).contiguous() if t.dim() > 2 else t.contiguous() for t in tensors)
+
+
+def _by_channel(*tensors):
+    """(rows, 3, chan) or (rows, 9, chan) as (rows, chan, 3, ..)"""
+    return tuple(t if t.dim() == 2 else t.transpose(1, 2).reshape(t.shape[0], -1, *([3] if t.shape[1] == 3 else [3, 3])).contiguous()
+                 for t in tensors)
+
+
+def _as_rows(P0, S1, S2):
+    """P0, S1, S2 as plain rows, one per (row, component)"""
+    return P0.flatten(1), S1.reshape(-1, 5 * S1.shape[-1]), S2.reshape(-1, 5 * S2.shape[-1])
 
 
 class _MessageProducts(torch.autograd.Function):
-    """The same with everything between the node operands and the per-node sums folded into kernels.  Forward: the
-    inference kernel of the layer (mg_bee_message: filters formed in registers, node rows gathered at the destination,
+    """The same with everything between the node operands and the per-node sums folded into kernels.  by_label: operands
+    and 13 results as in the plain formulation; else v_node (nodes, 3, chan), d_node (nodes, 9, chan) and the results as the plain
+    rows of P0, S1, S2 (ops.bee_message), which the output linears of a rank read as one, and then bounds of the row maxima of
+    |S1|, |S2| per node and of |P0| (empty when not known).
+    Forward: the inference kernel of the layer (mg_bee_message: filters formed in registers, node rows gathered at the destination,
     products summed over the edges of a node; only the three scalar products are stored per edge) when `enc_source`
     = (the 8 radial functions, weight and bias of the encoding linear) is given, else the indexed product kernel and
     segment sums.  Backward: one kernel walks the edges of a source node with the gradients of its sums in registers and
@@ -926,61 +942,142 @@ class _MessageProducts(torch.autograd.Function):
     differentiates the plain formulation instead."""
 
     @staticmethod
-    def forward(ctx, a_node, v_node, d_node, enc, rh, by_dst, by_src, enc_source):
-        from .ops import BEE_ORDER
-        ctx.by_dst, ctx.by_src = by_dst, by_src
+    def forward(ctx, a_node, v_node, d_node, enc, rh, by_dst, by_src, enc_source, by_label):
+        ctx.by_dst, ctx.by_src, ctx.by_label = by_dst, by_src, by_label
+        ctx.set_materialize_grads(False)
         a_node, v_node, d_node, enc, rh = (t.contiguous() for t in (a_node, v_node, d_node, enc, rh))
         ctx.save_for_backward(a_node, v_node, d_node, enc, rh)
         ctx.save_for_forward(a_node, v_node, d_node, enc, rh)
         N, C = a_node.shape
+        left = a_node, v_node, d_node
+        node_max = edge_max = enc.new_empty(0)
         if enc_source is not None:
             enc8, W, b = enc_source
             b = b if b is not None else torch.zeros(C, dtype=torch.float32, device=enc.device)
-            P0, S1, S2 = ops.bee_message(by_src.row_ptr, by_dst.index, rh, enc8.contiguous(), a_node,
-                                         v_node.transpose(1, 2).contiguous(),
-                                         d_node.reshape(N, C, 9).transpose(1, 2).contiguous(),
-                                         W.detach().contiguous(), b.detach().contiguous())
-            by_label = {lab: P0[:, k].contiguous() for k, lab in enumerate(("000", "110", "220"))}
-            for k, lab in enumerate(_S1_LABELS):
-                by_label[lab] = S1[:, :, k].transpose(1, 2).contiguous()
-            for k, lab in enumerate(_S2_LABELS):
-                by_label[lab] = S2[:, :, k].transpose(1, 2).contiguous().reshape(N, C, 3, 3)
-            return tuple(by_label[lab] for lab in BEE_ORDER)
-        phi_v, phi_d = ops.bee_edge_filters_fwd(enc, rh)
-        prods = ops.bee_fwd_indexed(a_node, v_node, d_node, by_dst.index, enc, phi_v, phi_d)
-        return tuple(p if lab[2] == "0" else ops.segment_sum_csr(p, by_src.row_ptr, by_src.n_rows)
-                     for lab, p in zip(BEE_ORDER, prods))
+            *stacked, node_max, edge_max = ops.bee_message(by_src.row_ptr, by_dst.index, rh, enc8.contiguous(),
+                                                           *(_by_component(*left) if by_label else left),
+                                                           W.detach().contiguous(), b.detach().contiguous(), want_node_max=True)
+            if by_label:
+                return ops.unstack_products(*stacked)
+        else:
+            phi_v, phi_d = ops.bee_edge_filters_fwd(enc, rh)
+            prods = ops.bee_fwd_indexed(*(left if by_label else (t.contiguous() for t in _by_channel(*left))), by_dst.index, enc,
+                                        phi_v, phi_d)
+            prods = tuple(p if lab[2] == "0" else ops.segment_sum_csr(p, by_src.row_ptr, by_src.n_rows)
+                          for lab, p in zip(ops.BEE_ORDER, prods))
+            if by_label:
+                return prods
+            stacked = ops.stack_products(prods)
+        ctx.mark_non_differentiable(node_max, edge_max)
+        return (*_as_rows(*stacked), node_max, edge_max)
 
     @staticmethod
     def jvp(ctx, a_t, v_t, d_t, enc_t, rh_t, *_):
         """Forward mode through the plain formulation: the products are bilinear in (node operands, edge filters), so
         the tangent is P(gathered tangents, filters) + P(gathered operands, the filters' tangent), summed per node
-        like the products themselves (an operand without a tangent arrives as zeros)."""
-        from .ops import BEE_ORDER
-        a_node, v_node, d_node, enc, rh = ctx.saved_tensors
-        by_dst, by_src = ctx.by_dst, ctx.by_src
-        gather = lambda ts: [gl._Gather.apply(t, by_dst) for t in ts]
+        like the products themselves."""
+        *left, enc, rh = ctx.saved_tensors
+        left_t = [torch.zeros_like(t) if g is None else g for g, t in zip((a_t, v_t, d_t), left)]
+        enc_t, rh_t = (torch.zeros_like(t) if g is None else g for g, t in zip((enc_t, rh_t), (enc, rh)))
+        by_dst, by_src, by_label = ctx.by_dst, ctx.by_src, ctx.by_label
+        gather = lambda ts: [gl._Gather.apply(t.contiguous(), by_dst) for t in (ts if by_label else _by_channel(*ts))]
         phi_v, phi_d = _EdgeFilters.apply(enc, rh)
         phi_v_t, phi_d_t = _edge_filters_tangent(enc, rh, enc_t, rh_t)
-        left = Bee.apply(*gather((a_t, v_t, d_t)), enc, phi_v, phi_d)
-        right = Bee.apply(*gather((a_node, v_node, d_node)), enc_t.contiguous(), phi_v_t.contiguous(), phi_d_t.contiguous())
-        prods = [a + b for a, b in zip(left, right)]
-        return tuple(p if lab[2] == "0" else gl._ScatterSum.apply(p.contiguous(), by_src) for lab, p in zip(BEE_ORDER, prods))
+        prods = [a + b for a, b in zip(Bee.apply(*gather(left_t), enc, phi_v, phi_d),
+                                       Bee.apply(*gather(left), enc_t.contiguous(), phi_v_t.contiguous(), phi_d_t.contiguous()))]
+        prods = tuple(p if lab[2] == "0" else gl._ScatterSum.apply(p.contiguous(), by_src) for lab, p in zip(ops.BEE_ORDER, prods))
+        return prods if by_label else (*_as_rows(*ops.stack_products(prods)), None, None)
 
     @staticmethod
     def backward(ctx, *dys):
-        saved, by_dst, by_src = ctx.saved_tensors, ctx.by_dst, ctx.by_src
+        saved, by_dst, by_src, by_label = ctx.saved_tensors, ctx.by_dst, ctx.by_src, ctx.by_label
         need = ctx.needs_input_grad
         if torch.is_grad_enabled():
             with torch.enable_grad():
                 leaves = [t if t.requires_grad else t.detach().requires_grad_() for t in saved]
-                out = _message_products_plain(*leaves, by_dst, by_src)
-                grads = torch.autograd.grad(out, leaves, dys, create_graph=True)
-            return tuple(g if nd else None for g, nd in zip(grads, need)) + (None, None, None)
+                out = _message_products_plain(*(leaves[:3] if by_label else _by_channel(*leaves[:3])), *leaves[3:], by_dst, by_src)
+                out = out if by_label else _as_rows(*ops.stack_products(out))
+                out, dys = zip(*((o, g) for o, g in zip(out, dys) if g is not None))
+                grads = torch.autograd.grad(out, leaves, dys, create_graph=True, allow_unused=True)
+            return tuple(g if nd else None for g, nd in zip(grads, need)) + (None, None, None, None)
         *left, enc, rh = saved
-        d_l, d_enc, d_rh = ops.bee_message_bwd(left, enc, rh, [dy.contiguous() for dy in dys], by_src, by_dst, any(need[:3]),
-                                               need[3], need[4])
-        return tuple(d_l[k] if need[k] else None for k in range(3)) + (d_enc, d_rh, None, None, None)
+        N, C, E = left[0].shape[0], left[0].shape[1], enc.shape[0]
+        if by_label:
+            run = ops.bee_message_bwd
+            shapes = [(by_src.n_rows if lab[2] != "0" else E, C, *[3] * int(lab[2])) for lab in ops.BEE_ORDER]
+        else:
+            run, shapes = ops.bee_message_grad, ((E, 3, C), (by_src.n_rows, 3, 5, C), (by_src.n_rows, 9, 5, C))
+        dys = [enc.new_zeros(sh) if g is None else g.contiguous().reshape(sh) for g, sh in zip(dys, shapes)]
+        d_l, d_enc, d_rh = run(left, enc, rh, dys, by_src, by_dst, any(need[:3]), need[3], need[4])
+        return tuple(d_l[k] if need[k] else None for k in range(3)) + (d_enc, d_rh, None, None, None, None)
+
+
+class _NodeProducts(torch.autograd.Function):
+    """The 13 products of operands (rows, chan), (rows, 3, chan), (rows, 9, chan) as the plain rows of P0, P1, P2
+    (ops.bee_node_products), and bounds of the row maxima of all of them per row (empty when not known).  A recorded backward
+    pass differentiates the product function instead, forward mode is the product rule."""
+
+    @staticmethod
+    def forward(ctx, *operands):
+        operands = tuple(t.contiguous() for t in operands)
+        ctx.save_for_backward(*operands)
+        ctx.save_for_forward(*operands)
+        ctx.set_materialize_grads(False)
+        *stacked, node_max = ops.bee_node_products(*operands, want_node_max=True)
+        node_max = node_max if node_max is not None else operands[0].new_empty(0)
+        ctx.mark_non_differentiable(node_max)
+        return (*_as_rows(*stacked), node_max)
+
+    @staticmethod
+    def jvp(ctx, *tangents):
+        operands = ctx.saved_tensors
+        tangents = [torch.zeros_like(x) if t is None else t for t, x in zip(tangents, operands)]
+        left, right = _NodeProducts.apply(*tangents[:3], *operands[3:]), _NodeProducts.apply(*operands[:3], *tangents[3:])
+        return (*(a + b for a, b in zip(left[:3], right[:3])), None)
+
+    @staticmethod
+    def backward(ctx, *dys):
+        operands, need = ctx.saved_tensors, ctx.needs_input_grad
+        if torch.is_grad_enabled():
+            with torch.enable_grad():
+                leaves = [t if t.requires_grad else t.detach().requires_grad_() for t in operands]
+                out = _as_rows(*ops.stack_products(Bee.apply(*_by_channel(*leaves))))
+                out, dys = zip(*((o, g) for o, g in zip(out, dys) if g is not None))
+                grads = torch.autograd.grad(out, leaves, dys, create_graph=True, allow_unused=True)
+        else:
+            N, C = operands[0].shape
+            shapes = (N, 3, C), (N, 3, 5, C), (N, 9, 5, C)
+            grads = ops.bee_node_products_grad(operands, [operands[0].new_zeros(sh) if g is None else g.contiguous()
+                                                          for g, sh in zip(dys, shapes)])
+        return tuple(g if nd else None for g, nd in zip(grads, need))
+
+
+def _component_rows(x):
+    """(.., chan, 3, ..) of rank 1 or 2 as plain rows, one per (row, component)"""
+    return x.flatten(2).transpose(1, 2).reshape(-1, x.shape[1])
+
+
+def _linear_by_component(lin, rank, rows):
+    """A TensLinear of rank 0, 1 or 2 on the plain rows of x -> (rows of x, chan) or (rows of x, 3^rank, chan)."""
+    y = tensor_linear(0, lin.W, rows, sequential=torch.is_grad_enabled())
+    return y if rank == 0 else y.reshape(-1, 3 ** rank, y.shape[-1])
+
+
+def _linears_of_rank(mod, rank, P, bound, rows):
+    """The output linears of one rank, summed: one linear on the plain rows P, whose weights lie side by side.  Returns
+    (rows, dim), (rows, dim, 3) or (rows, dim, 3, 3)."""
+    W = torch.cat([getattr(mod, f"Y_{lab}").W for lab in ops.STACKED[rank]], dim=1)
+    if not bound.numel():
+        bound = None
+    elif rank:
+        bound = bound.repeat_interleave(3 ** rank, dim=0)
+    y = tensor_linear(0, W, P, x_bound=bound, sequential=torch.is_grad_enabled())
+    return y if rank == 0 else y.reshape(rows, 3 ** rank, -1).transpose(1, 2).reshape(rows, -1, *[3] * rank)
+
+
+def _plain_linears(mod, operands):
+    """True when calling the module's tensor linears (the operands' and Y_*) does what TensLinear.forward does and nothing else."""
+    return all(plain_call(getattr(mod, name), TensLinear) for name in (*operands, *(f"Y_{lab}" for lab in ops.BEE_ORDER)))
 
 
 def message_products(graph, a_node, v_node, d_node, enc, rh, enc_source=None):
@@ -991,7 +1088,7 @@ def message_products(graph, a_node, v_node, d_node, enc, rh, enc_source=None):
     flat = [gl._flat_nodes(graph, t) for t in (a_node, v_node, d_node)]
     enc, rh = enc.contiguous(), rh.contiguous()
     if ops.bee_indexed_supported(enc.size(1)) and all(t.data_ptr() % 16 == 0 for t in flat + [enc]):
-        return _MessageProducts.apply(*flat, enc, rh, graph.by_dst, graph.by_src, enc_source)
+        return _MessageProducts.apply(*flat, enc, rh, graph.by_dst, graph.by_src, enc_source, True)
     return _message_products_plain(*flat, enc, rh, graph.by_dst, graph.by_src)
 
 
@@ -1042,6 +1139,17 @@ def bee_messages(msg, graph, r_ij, x_a, x_v, x_d):
     # The output linears of the vector and rank-2 channels have no bias and nothing nonlinear follows them before the
     # sum over edges, so they commute with it: the products are summed per node first and the ten linears run on N
     # rows, not E (the reference applies them per edge).  The scalar channel goes through an MLP per edge.
+    B, N = x_a.shape[:2]
+    if _plain_linears(msg, ("L0", "L1", "L2")) and ops.bee_indexed_supported(enc.size(1)):
+        a, v, d = (gl._flat_nodes(graph, t) for t in (x_a, x_v, x_d))
+        nodes = [_linear_by_component(lin, k, x)
+                 for k, (lin, x) in enumerate(zip((msg.L0, msg.L1, msg.L2), (a, _component_rows(v), _component_rows(d))))]
+        P0, S1, S2, node_max, edge_max = _MessageProducts.apply(*nodes, enc, rh, graph.by_dst, graph.by_src,
+                                                                (enc8.detach(), msg.lin_enc.weight, msg.lin_enc.bias), False)
+        psi_a = _linears_of_rank(msg, 0, P0, edge_max, None)
+        sums = [_linears_of_rank(msg, k, S, node_max, B * N) for k, S in ((1, S1), (2, S2))]
+        psi_a = psi_a + mlp_leaky(msg.mlp_a, psi_a)
+        return (mul(gl.edges_reduce_src(graph, psi_a), 0.1), *(mul(t.reshape(B, N, *t.shape[1:]), 0.1) for t in sums))
     prods = message_products(graph, msg.L0(x_a), msg.L1(x_v), msg.L2(x_d), enc, rh,
                              enc_source=(enc8.detach(), msg.lin_enc.weight, msg.lin_enc.bias))
     from .ops import BEE_ORDER
@@ -1074,7 +1182,14 @@ def self_tens_prods(mod, x_a, x_v, x_d):
     *rest, dim_a = x_a.shape
     dim_v, dim_d = x_v.shape[-2], x_d.shape[-3]
     a, v, d = x_a.reshape(-1, dim_a), x_v.reshape(-1, dim_v, 3), x_d.reshape(-1, dim_d, 3, 3)
-    prods = Bee.apply(mod.L0(a), mod.L1(v), mod.L2(d), mod.R0(a), mod.R1(v), mod.R2(d))
-    y_a, y_v, y_d = apply_tens_prod_submodules(mod, prods)
+    if _plain_linears(mod, ("L0", "L1", "L2", "R0", "R1", "R2")):
+        rows = a, _component_rows(v), _component_rows(d)
+        operands = [_linear_by_component(lin, k, x) for side in ((mod.L0, mod.L1, mod.L2), (mod.R0, mod.R1, mod.R2))
+                    for k, (lin, x) in enumerate(zip(side, rows))]
+        *stacked, node_max = _NodeProducts.apply(*operands)
+        y_a, y_v, y_d = (_linears_of_rank(mod, k, P, node_max, a.shape[0]) for k, P in enumerate(stacked))
+    else:
+        prods = Bee.apply(mod.L0(a), mod.L1(v), mod.L2(d), mod.R0(a), mod.R1(v), mod.R2(d))
+        y_a, y_v, y_d = apply_tens_prod_submodules(mod, prods)
     return (tens_group_norm(mod.gn_a, y_a.reshape(*rest, dim_a)), tens_group_norm(mod.gn_v, y_v.reshape(*rest, dim_v, 3)),
             tens_group_norm(mod.gn_d, y_d.reshape(*rest, dim_d, 3, 3)))

@@ -18,6 +18,8 @@ _lib = L.load()
 _ext = L.load_torch_ext()       # the C++ host side of the hot calls (csrc/torch_ops.cpp)
 
 BEE_ORDER = ("000", "110", "220", "011", "101", "121", "211", "022", "202", "112", "222", "111", "212")
+# the same by rank, in the order of P0, S1, S2 of bee_message
+STACKED = (("000", "110", "220"), ("011", "101", "121", "211", "111"), ("022", "202", "112", "222", "212"))
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
@@ -575,12 +577,39 @@ def bee_bwd_indexed(side, o_0, o_1, o_2, o_index, dys, dy_index, rows):
     return d
 
 
-def bee_message_bwd(left, enc, rh, dys, by_src, by_dst, want_left, want_enc, want_rh):
-    """Gradients of the 13 products of the node operands `left`, read at the edges' destinations, with the edge filters made
-    of enc (edges, chan) and rh (edges, 3): ([d_l0, d_l1, d_l2] or [], d_enc or None, d_rh or None).  dys: one row per edge
-    for the scalar products, one per source node for the others (their sums over its edges)."""
-    return _ext.bee_message_bwd(list(left), enc, rh, list(dys), by_src.row_ptr, by_dst.index, by_dst.row_ptr, by_dst.perm,
+def bee_message_grad(left, enc, rh, d_products, by_src, by_dst, want_left, want_enc, want_rh):
+    """Gradients of bee_message for the node operands `left` (nodes, chan), (nodes, 3, chan), (nodes, 9, chan), read at the edges'
+    destinations, and for enc (edges, chan) and rh (edges, 3), which the edge filters are made of: ([d_l0, d_l1, d_l2] or
+    [], d_enc or None, d_rh or None).  d_products: those of P0, S1 and S2."""
+    return _ext.bee_message_bwd(list(left), enc, rh, list(d_products), by_src.row_ptr, by_dst.index, by_dst.row_ptr, by_dst.perm,
                                 bool(want_left), bool(want_enc), bool(want_rh))
+
+
+def bee_message_bwd(left, enc, rh, dys, by_src, by_dst, want_left, want_enc, want_rh):
+    """bee_message_grad with the operands and their gradients as (nodes, chan, 3, ..) and those of the 13 products one by one, in
+    BEE_ORDER: one row per edge for the scalar products, one per source node for the others (their sums over its edges)."""
+    n, chan = left[0].shape
+    by_comp = [left[0]] + [t.reshape(n, chan, -1).transpose(1, 2).contiguous() for t in left[1:]]
+    d_left, d_enc, d_rh = bee_message_grad(by_comp, enc, rh, stack_products(dys), by_src, by_dst, want_left, want_enc, want_rh)
+    return [d.transpose(1, 2).reshape(t.shape) if d.dim() == 3 else d for d, t in zip(d_left, left)], d_enc, d_rh
+
+
+def stack_products(prods):
+    """The 13 products (rows, chan, 3, ..) in BEE_ORDER as P0 (rows, 3, chan), S1 (rows, 3, 5, chan), S2 (rows, 9, 5, chan) of
+    bee_message and bee_node_products (the scalar ones may have rows of their own)."""
+    of = dict(zip(BEE_ORDER, prods))
+    stacked = [torch.stack([of[lab].flatten(2) if lab[2] != "0" else of[lab] for lab in labels], dim=1) for labels in STACKED]
+    return stacked[0], stacked[1].permute(0, 3, 1, 2).contiguous(), stacked[2].permute(0, 3, 1, 2).contiguous()
+
+
+def unstack_products(P0, S1, S2):
+    """The 13 products (rows, chan, 3, ..) in BEE_ORDER, contiguous, from P0, S1, S2."""
+    of = {lab: P0[:, k].contiguous() for k, lab in enumerate(STACKED[0])}
+    for rank, S in ((1, S1), (2, S2)):
+        for k, lab in enumerate(STACKED[rank]):
+            p = S[:, :, k].transpose(1, 2).contiguous()
+            of[lab] = p.reshape(*p.shape[:2], *[3] * rank)
+    return tuple(of[lab] for lab in BEE_ORDER)
 
 
 def bee_bwl(r_0, r_1, r_2, *dys):
@@ -1313,6 +1342,22 @@ def bee_node_products(l0, l1, l2, r0, r1, r2, want_node_max=False):
             L.check(_lib.mg_bee_node_products(N, chan, _p(l0), _p(l1), _p(l2), _p(r0), _p(r1), _p(r2), _p(P0), _p(P1),
                                               _p(P2), _p(node_max), _stream()))
     return (P0, P1, P2, node_max) if want_node_max else (P0, P1, P2)
+
+
+def bee_node_products_grad(operands, d_products):
+    """The gradients of bee_node_products (float32) for its six operands from those of P0, P1, P2."""
+    l0 = operands[0]
+    for t in (*operands, *d_products):
+        _check_input(t, "operand or gradient")
+    N, chan = int(l0.size(0)), int(l0.size(1))
+    if [t.numel() for t in operands] != 2 * [N * chan, 3 * N * chan, 9 * N * chan]:
+        raise RuntimeError("operands must be (nodes, chan), (nodes, 3, chan), (nodes, 9, chan)")
+    if [t.numel() for t in d_products] != [3 * N * chan, 15 * N * chan, 45 * N * chan]:
+        raise RuntimeError("gradients must have the sizes of P0, P1, P2")
+    with _on(l0.device):
+        grads = [torch.empty_like(t) for t in operands]
+        L.check(_lib.mg_bee_node_products_grad(N, chan, *[_p(t) for t in (*operands, *d_products, *grads)], _stream()))
+    return grads
 
 
 def bf16_rowsum_supported(rows, dim_in, dim_out):
