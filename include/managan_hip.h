@@ -400,6 +400,32 @@ typedef struct mg_mlp_f16x2_grad {
 int mg_mlp_f16x2_supported(int dim_in, int dim);      /* returns 0 / 1, not a status */
 int mg_mlp_f16x2_forward(const mg_mlp_f16x2* args /* host */, mg_stream_t stream);
 int mg_mlp_f16x2_adjoint(const mg_mlp_f16x2_grad* args /* host */, mg_stream_t stream);
+/* Linear, LeakyReLU(0.1), Linear, LeakyReLU(0.1), Linear (archs/diffuser_atoms15.py:98-110) under differentiation, as the above:
+ * x (rows, dim_in), hidden layers of `dim` columns, y (rows, dim_out), all of them multiples of 32 up to 512.  Kept per hidden layer: h =
+ * LeakyReLU(z), whose sign is that of z, and the row maxima of |h|.  A row's results do not depend on the other rows. */
+typedef struct mg_mlp_leaky_f16x2 {
+    const float* x;
+    long rows;
+    int dim_in, dim, dim_out;
+    const void* packed_W[3];
+    const float* bias[3];
+    float* y;
+    float *h[2], *h_rowmax[2];
+    float* x_rowmax;
+} mg_mlp_leaky_f16x2;
+typedef struct mg_mlp_leaky_f16x2_grad {
+    const float* dy;
+    long rows;
+    int dim_in, dim, dim_out;
+    const void* packed_Wt[3];
+    const float* h[2];
+    float *dz[2], *dz_rowmax[2];
+    float* dx;
+    float* dy_rowmax;
+} mg_mlp_leaky_f16x2_grad;
+int mg_mlp_leaky_f16x2_supported(int dim_in, int dim, int dim_out);      /* returns 0 / 1, not a status */
+int mg_mlp_leaky_f16x2_forward(const mg_mlp_leaky_f16x2* args /* host */, mg_stream_t stream);
+int mg_mlp_leaky_f16x2_adjoint(const mg_mlp_leaky_f16x2_grad* args /* host */, mg_stream_t stream);
 /* The nonlinear layers of an MLP whose result is only needed summed over the rows of segments (archs/diffuser_atoms15.py:98-110
  * under edges_reduce_src, :244-246): out[s] = sum over the rows r of segment s of f(W2 f(W1 x[r] + b1) + b2), f = LeakyReLU(0.1),
  * x (rows, dim_in), both layers `dim` wide, out (n_out, dim).  Rows are sorted by segment (seg ascending, row_ptr its CSR form);

@@ -216,11 +216,14 @@ __device__ __forceinline__ void split_rows(_Float16* xh, float* row_max, int K, 
     }
 }
 
-// DUAL: the 32 rows of a block are 16 values and their 16 tangents
-template <int MI, int NI, int MODE, bool DUAL>
+// DUAL: the 32 rows of a block are 16 values and their 16 tangents.  LEAKY: LeakyReLU(0.1) in SiLU's place, whose input need not be
+// kept (h has its sign), and a last layer of N columns.
+template <int MI, int NI, int MODE, bool DUAL, bool LEAKY = false>
 __global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const MlpArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     static_assert(!DUAL || MI == 1, "one block of values and tangents");
+    static_assert(!LEAKY || (!DUAL && MODE != kInfer), "LeakyReLU: values under differentiation");
+    constexpr bool kTail = MODE == kAdjoint || LEAKY;              // the last layer is not O columns wide
     constexpr int TM = 32 * MI, kRows = DUAL ? 16 : TM;
     constexpr int kSums = MI * NI == 1 ? 2 : 1;                    // (what 128 registers hold)
     const int O = a.O, widest = a.K > O ? a.K : O;
@@ -255,7 +258,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const
         __syncthreads();                                           // (row_max is written again below)
     }
 
-    constexpr int kFull = MODE == kAdjoint ? 2 : 3;                // layers with O columns
+    constexpr int kFull = kTail ? 2 : 3;                           // layers with O columns
     int K = a.K;
 #pragma unroll 1
     for (int l = 0; l < kFull; l++) {
@@ -291,7 +294,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const
             }
         }
 
-        const bool last = MODE != kAdjoint && l == kFull - 1;
+        const bool last = !kTail && l == kFull - 1;
         float mx[MI];
 #pragma unroll
         for (int mi = 0; mi < MI; mi++) mx[mi] = 0.f;
@@ -335,6 +338,19 @@ __global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const
                         for (int k = 0; k < 2; k++)
 #pragma unroll
                             for (int i = 0; i < 4; i++) v[k][i] = v[k][i] * __builtin_amdgcn_rcpf(1.0f + __expf(-v[k][i]));
+                    } else if constexpr (LEAKY) {
+#pragma unroll
+                        for (int k = 0; k < 2; k++) {
+                            float h[4] = {1.f, 1.f, 1.f, 1.f};
+                            if (MODE == kAdjoint) {
+                                const float4 h4 = *reinterpret_cast<const float4*>(a.z_in[l] + at + 16 * k);
+                                h[0] = h4.x; h[1] = h4.y; h[2] = h4.z; h[3] = h4.w;
+                            }
+#pragma unroll
+                            for (int i = 0; i < 4; i++)
+                                v[k][i] = (MODE == kAdjoint ? h[i] : v[k][i]) > 0.f ? v[k][i] : 0.1f * v[k][i];
+                        }
+                        put(a.h[l]);
                     } else if constexpr (MODE == kTrain) {
                         put(a.z[l]);
 #pragma unroll
@@ -387,7 +403,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const
 
         // the next layer's rows: their maxima, then their pieces in the place of this layer's
         const bool marked = has_marks(a.inv[l + 1 < kFull ? l + 1 : kFull - 1], O, lane) ||
-                            (MODE == kAdjoint && l + 1 == kFull && a.y && has_marks(a.inv[2], a.N, lane));
+                            (kTail && l + 1 == kFull && a.y && has_marks(a.inv[2], a.N, lane));
 #pragma unroll
         for (int mi = 0; mi < MI; mi++) {
             mx[mi] = fmaxf(mx[mi], __shfl_xor(mx[mi], 32));
@@ -419,8 +435,8 @@ __global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const
         __syncthreads();
     }
 
-    // adjoint: the gradient of x, O -> N columns, 32 to a wave at a time
-    if constexpr (MODE == kAdjoint) {
+    // adjoint: the gradient of x; O -> N columns, 32 to a wave at a time
+    if constexpr (kTail) {
         if (!a.y) return;
         const int N = a.N, x_lo = TM * O;
         const long w_lo = (long)pad256(N) * O;
@@ -433,20 +449,23 @@ __global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const
             for (int mi = 0; mi < MI; mi++) {
                 if (!live(mi)) continue;
                 float* out = a.y + row_of(mi, m) * N + 32 * nb + 4 * G;
+                const float* bias = MODE == kAdjoint ? nullptr : a.bias[2];
                 if (odd[mi]) {
 #pragma unroll 1
                     for (int q = 0; q < 16; q++) {
                         const int c = 8 * (q / 4) + q % 4, n = 32 * nb + 4 * G + c;
-                        out[c] = lds_row_in_fp32(xh + mi * 32 * O, x_lo, m, a.planes[2], w_lo, n, O, inv[n]);
+                        out[c] = lds_row_in_fp32(xh + mi * 32 * O, x_lo, m, a.planes[2], w_lo, n, O, inv[n]) + (bias ? bias[n] : 0.f);
                     }
                     continue;
                 }
 #pragma unroll
                 for (int t = 0; t < 4; t++) {
                     const float4 iw = *reinterpret_cast<const float4*>(inv + 32 * nb + 8 * t + 4 * G);
+                    float4 b = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (bias) b = *reinterpret_cast<const float4*>(bias + 32 * nb + 8 * t + 4 * G);
                     *reinterpret_cast<float4*>(out + 8 * t) =
-                        make_float4(acc[mi][0][4 * t] * isx[mi] * iw.x, acc[mi][0][4 * t + 1] * isx[mi] * iw.y,
-                                    acc[mi][0][4 * t + 2] * isx[mi] * iw.z, acc[mi][0][4 * t + 3] * isx[mi] * iw.w);
+                        make_float4(acc[mi][0][4 * t] * isx[mi] * iw.x + b.x, acc[mi][0][4 * t + 1] * isx[mi] * iw.y + b.y,
+                                    acc[mi][0][4 * t + 2] * isx[mi] * iw.z + b.z, acc[mi][0][4 * t + 3] * isx[mi] * iw.w + b.w);
                 }
             }
         }
@@ -626,9 +645,9 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 4) mlp_rowsum_f16x2_kernel(con
     *to = sum;
 }
 
-template <int MI, int NI, int MODE, bool DUAL>
+template <int MI, int NI, int MODE, bool DUAL, bool LEAKY = false>
 int launch(const MlpArgs& a, hipStream_t st) {
-    const auto kernel = mlp_f16x2_kernel<MI, NI, MODE, DUAL>;
+    const auto kernel = mlp_f16x2_kernel<MI, NI, MODE, DUAL, LEAKY>;
     const int widest = a.K > a.O ? a.K : a.O;
     const size_t lds = (size_t)32 * MI * widest * 4 + (kMaxWaves / NI * 32 * MI + kMaxDim) * sizeof(float);
     // more than 64 KB of dynamic LDS has to be asked for (per device, so on every call)
@@ -655,6 +674,15 @@ int choose(const MlpArgs& a, bool dual, hipStream_t st) {
         if (a.O > 256 && a.O % 64 == 0 && tiles > 256) return dual ? launch<1, 2, MODE, true>(a, st) : launch<1, 2, MODE, false>(a, st);
         return dual ? launch<1, 1, MODE, true>(a, st) : launch<1, 1, MODE, false>(a, st);
     }
+}
+
+// Two column blocks to a wave, so that two workgroups share a CU, where the width has them: by the width alone and not by the rows as
+// above, since the slope at zero should not depend on how many rows a call has.  127 000 rows, 256 -> 512 -> 512 -> 256: 0.57 ms, the
+// adjoint 0.72 (weights out of the L2 at 14 TB/s, 1.3 GB of kept rows); four linears, the activations, their derivatives and the row
+// maxima in passes of their own took 0.4 ms more of a training step with two such MLPs each way.
+template <int MODE>
+int launch_leaky(const MlpArgs& a, hipStream_t st) {
+    return a.O % 64 == 0 ? launch<1, 2, MODE, false, true>(a, st) : launch<1, 1, MODE, false, true>(a, st);
 }
 
 int fill(MlpArgs& a, const void* const* packed, int K, int O, int N) {
@@ -731,6 +759,60 @@ int mg_mlp_f16x2_adjoint(const mg_mlp_f16x2_grad* p, mg_stream_t stream) {
     MG_REQUIRE(fill(a, packed, a.O, a.O, a.N) && packed[0] && packed[1] && (packed[2] || !a.y) && a.x && aligned16(a.x) && aligned16(a.y),
                "mg_mlp_f16x2_adjoint: null or unaligned pointer");
     return choose<kAdjoint>(a, p->dual, (hipStream_t)stream);
+}
+
+int mg_mlp_leaky_f16x2_supported(int dim_in, int dim, int dim_out) {
+    return mg_mlp_f16x2_supported(dim_in, dim) && mg_mlp_f16x2_supported(dim_out, dim);
+}
+
+int mg_mlp_leaky_f16x2_forward(const mg_mlp_leaky_f16x2* p, mg_stream_t stream) {
+    MG_REQUIRE(p != nullptr && p->rows >= 0 && mg_mlp_leaky_f16x2_supported(p->dim_in, p->dim, p->dim_out),
+               "mg_mlp_leaky_f16x2_forward: dimensions must be multiples of 32 up to %d", kMaxDim);
+    if (p->rows == 0) return MG_OK;
+    MlpArgs a{};
+    a.x = p->x;
+    a.R = p->rows;
+    a.K = p->dim_in;
+    a.O = p->dim;
+    a.N = p->dim_out;
+    a.y = p->y;
+    a.x_max = p->x_rowmax;
+    for (int l = 0; l < 3; l++) {
+        a.bias[l] = p->bias[l];
+        MG_REQUIRE(p->packed_W[l] && (!p->bias[l] || aligned16(p->bias[l])), "mg_mlp_leaky_f16x2_forward: null or unaligned weight or bias");
+        if (l == 2) break;
+        a.h[l] = p->h[l];
+        a.h_max[l] = p->h_rowmax[l];
+        MG_REQUIRE(a.h[l] && a.h_max[l] && aligned16(a.h[l]), "mg_mlp_leaky_f16x2_forward: null or unaligned pointer");
+    }
+    MG_REQUIRE(fill(a, p->packed_W, a.K, a.O, a.N) && a.x && a.y && aligned16(a.x) && aligned16(a.y),
+               "mg_mlp_leaky_f16x2_forward: null or unaligned pointer");
+    return launch_leaky<kTrain>(a, (hipStream_t)stream);
+}
+
+int mg_mlp_leaky_f16x2_adjoint(const mg_mlp_leaky_f16x2_grad* p, mg_stream_t stream) {
+    MG_REQUIRE(p != nullptr && p->rows >= 0 && mg_mlp_leaky_f16x2_supported(p->dim_in, p->dim, p->dim_out),
+               "mg_mlp_leaky_f16x2_adjoint: dimensions must be multiples of 32 up to %d", kMaxDim);
+    if (p->rows == 0) return MG_OK;
+    MlpArgs a{};
+    a.x = p->dy;
+    a.R = p->rows;
+    a.K = p->dim_out;
+    a.O = p->dim;
+    a.N = p->dim_in;
+    a.y = p->dx;
+    a.x_max = p->dy_rowmax;
+    for (int l = 0; l < 2; l++) {                                  // met in reverse
+        a.z_in[l] = p->h[1 - l];
+        a.h[l] = p->dz[1 - l];
+        a.h_max[l] = p->dz_rowmax[1 - l];
+        MG_REQUIRE(a.z_in[l] && a.h[l] && a.h_max[l] && aligned16(a.z_in[l]) && aligned16(a.h[l]),
+                   "mg_mlp_leaky_f16x2_adjoint: null or unaligned pointer");
+    }
+    const void* packed[3] = {p->packed_Wt[2], p->packed_Wt[1], p->packed_Wt[0]};
+    MG_REQUIRE(fill(a, packed, a.K, a.O, a.N) && packed[0] && packed[1] && (packed[2] || !a.y) && a.x && aligned16(a.x) && aligned16(a.y),
+               "mg_mlp_leaky_f16x2_adjoint: null or unaligned pointer");
+    return launch_leaky<kAdjoint>(a, (hipStream_t)stream);
 }
 
 int mg_mlp_leaky_rowsum_f16x2_workspace_bytes(long rows, int dim, size_t* bytes) {

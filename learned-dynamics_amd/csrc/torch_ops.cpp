@@ -978,6 +978,99 @@ std::tuple<OptTensor, OptTensor, Tensors> mlp_silu_bwd(const at::Tensor& g, cons
     return {on_storage(*g_x, 0, x.sizes()), second_half(*g_x, x.sizes(), dual), params};
 }
 
+// x W_d^T + the three layers with LeakyReLU(0.1) between them; W: the layers' weights, then W_d.  From the row count at which plain
+// linears leave the fp32 kernel, for every size: the slope at zero should not depend on it.
+bool mlp_leaky_takes(const at::Tensor& x, const Tensors& W, const Tensors& b) {
+    if (mg_get_linear_mode() != kModeF16x2 || x.dim() != 2 || x.size(0) < 256 || W.size() != 4 || b.size() != 3) return false;
+    for (const at::Tensor& t : W)
+        if (!t.is_cuda() || t.scalar_type() != at::kFloat || t.dim() != 2 || !packs_f16x2(t)) return false;
+    const int64_t K = W[0].size(1), O = W[0].size(0), N = W[2].size(0);
+    if (x.size(1) != K || W[1].size(0) != O || W[1].size(1) != O || W[2].size(1) != O || W[3].size(0) != N || W[3].size(1) != K) return false;
+    for (int l = 0; l < 3; l++)
+        if (!b[l].is_cuda() || b[l].scalar_type() != at::kFloat || !b[l].is_contiguous() || b[l].numel() != W[l].size(0)) return false;
+    return x.is_cuda() && x.scalar_type() == at::kFloat && x.is_contiguous() && aligned16(x) && aligned_all(b) &&
+           mg_mlp_leaky_f16x2_supported((int)K, (int)O, (int)N);
+}
+
+// saved: row maxima of |x|, then h and its row maxima of either hidden layer
+std::tuple<at::Tensor, Tensors> mlp_leaky_fwd(const at::Tensor& x, const Tensors& W, const Tensors& b) {
+    TORCH_CHECK(mlp_leaky_takes(x, W, b), "mlp_leaky_fwd: sizes or types");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    pack_ahead({W[0], W[1], W[2], W[3], W[0].t(), W[1].t(), W[2].t(), W[3].t()});
+    const int64_t rows = x.size(0), dim = W[0].size(0);
+    mg_mlp_leaky_f16x2 a{};
+    at::Tensor y = floats(x, {rows, W[2].size(0)});
+    Tensors saved{floats(x, {rows, 1})}, planes;
+    for (int l = 0; l < 3; l++) {
+        planes.push_back(packed_f16x2(W[l], W[l].size(1)));
+        a.packed_W[l] = planes[l].data_ptr();
+        a.bias[l] = fp(b[l]);
+        if (l == 2) break;
+        saved.push_back(floats(x, {rows, dim}));
+        a.h[l] = fp(saved.back());
+        saved.push_back(floats(x, {rows, 1}));
+        a.h_rowmax[l] = fp(saved.back());
+    }
+    a.x = fp(x);
+    a.x_rowmax = fp(saved[0]);
+    a.rows = rows;
+    a.dim_in = (int)W[0].size(1);
+    a.dim = (int)dim;
+    a.dim_out = (int)W[2].size(0);
+    a.y = fp(y);
+    check(mg_mlp_leaky_f16x2_forward(&a, stream_of(x)));
+    run_f16x2(W[3], W[3].size(1), fp(x), rows, Bound{OptTensor(saved[0])}, OptTensor(), kActNone, true, 1, y, nullptr, true);
+    return {y, saved};
+}
+
+std::tuple<OptTensor, Tensors> mlp_leaky_bwd(const at::Tensor& g, const at::Tensor& x, const Tensors& W, const Tensors& saved,
+                                             bool want_x, bool want_params) {
+    check_input(g, "gradient");
+    TORCH_CHECK(W.size() == 4 && saved.size() == 5 && g.dim() == 2 && g.size(0) == x.size(0) && g.size(1) == W[2].size(0) && aligned16(g),
+                "mlp_leaky_bwd: sizes");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    const int64_t rows = x.size(0), dim = W[0].size(0);
+    mg_mlp_leaky_f16x2_grad a{};
+    at::Tensor dz[2], m[2], g_max = floats(x, {rows, 1});
+    OptTensor g_x;
+    Tensors planes;
+    for (int l = 0; l < 3; l++) {
+        planes.push_back(packed_f16x2(W[l].t(), W[l].size(0)));
+        a.packed_Wt[l] = planes[l].data_ptr();
+        if (l == 2) break;
+        dz[l] = floats(x, {rows, dim});
+        m[l] = floats(x, {rows, 1});
+        a.h[l] = fp(saved[1 + 2 * l]);
+        a.dz[l] = fp(dz[l]);
+        a.dz_rowmax[l] = fp(m[l]);
+    }
+    a.dy = fp(g);
+    a.dy_rowmax = fp(g_max);
+    if (want_x) {
+        g_x = floats(x, x.sizes());
+        a.dx = fp(*g_x);
+    }
+    a.rows = rows;
+    a.dim_in = (int)W[0].size(1);
+    a.dim = (int)dim;
+    a.dim_out = (int)W[2].size(0);
+    check(mg_mlp_leaky_f16x2_adjoint(&a, stream_of(x)));
+    if (want_x) run_f16x2(W[3].t(), W[3].size(0), fp(g), rows, Bound{OptTensor(g_max)}, OptTensor(), kActNone, true, 1, *g_x, nullptr, false);
+    Tensors params;
+    if (want_params) {
+        auto of = [&](const at::Tensor& dy, const at::Tensor& in, const at::Tensor& dy_bound, const at::Tensor& in_bound, bool bias) {
+            auto [dW, db] = rows_wgrad(dy, in, rows, bias, OptTensor(dy_bound), OptTensor(in_bound));
+            params.push_back(dW);
+            if (bias) params.push_back(*db);
+        };
+        of(dz[0], x, m[0], saved[0], true);
+        of(dz[1], saved[1], m[1], saved[2], true);
+        of(g, saved[3], g_max, saved[4], true);
+        of(g, x, g_max, saved[0], false);
+    }
+    return {g_x, params};
+}
+
 // enc, enc_t, row bounds of both, dir, dir_t
 std::tuple<at::Tensor, OptTensor, at::Tensor, at::Tensor, OptTensor> edge_encode_fwd(const at::Tensor& r, const OptTensor& r_t, int64_t n,
                                                                                      double rmax, double eps) {
@@ -1331,6 +1424,9 @@ void register_ops(pybind11::module_& m) {
     m.def("bee_message_bwd", &bee_message_bwd);
     m.def("mlp_silu_fwd", &mlp_silu_fwd);
     m.def("mlp_silu_bwd", &mlp_silu_bwd);
+    m.def("mlp_leaky_takes", &mlp_leaky_takes);
+    m.def("mlp_leaky_fwd", &mlp_leaky_fwd);
+    m.def("mlp_leaky_bwd", &mlp_leaky_bwd);
     m.def("edge_encode_fwd", &edge_encode_fwd);
     m.def("edge_encode_bwd", &edge_encode_bwd);
     m.def("combine_dual_fwd", &combine_dual_fwd);

@@ -291,12 +291,52 @@ def mlp_silu(mlp, x):
     return out if t is None else fwAD.make_dual(*out)
 
 
+class _MlpLeaky(torch.autograd.Function):
+    """bee_layers.MLP on rows: the layers as one kernel each way, the direct map added to their result.  params: weight and bias of
+    the three layers, then the direct map's weight."""
+
+    @staticmethod
+    def forward(ctx, x, *params):
+        y, rows = ops.mlp_leaky_fwd(x, params[0:6:2] + params[6:], params[1:6:2])
+        ctx.save_for_backward(x, *params, *(rows if any(ctx.needs_input_grad) else ()))
+        ctx.set_materialize_grads(False)
+        return y
+
+    @staticmethod
+    def backward(ctx, g):
+        x, *saved = ctx.saved_tensors
+        params, rows = saved[:7], saved[7:]
+        need = ctx.needs_input_grad
+        if g is None:
+            return (None,) * len(need)
+        if torch.is_grad_enabled():
+            return _recorded_gradients(lambda x, *p: (_mlp_leaky_rows(p, x),), (x, *params), need, (g,))
+        g = g.contiguous()
+        if g.data_ptr() % 16:
+            g = g.clone()
+        g_x, d_params = ops.mlp_leaky_bwd(g, x, params[0:6:2] + params[6:], rows, need[0], any(need[1:]))
+        return (g_x if need[0] else None,) + tuple(d if nd else None for d, nd in zip(d_params or [None] * 7, need[1:]))
+
+
+def _mlp_leaky_rows(params, x):
+    """The same out of differentiable pieces."""
+    W0, b0, W1, b1, W2, b2, Wd = params
+    z, b = tensor_linear(0, W0, x, bias=b0, want_bound=True, sequential=True)
+    z, b = tensor_linear(0, W1, F.leaky_relu(z, 0.1), bias=b1, x_bound=b, want_bound=True, sequential=True)
+    return tensor_linear(0, Wd, x, sequential=True) + tensor_linear(0, W2, F.leaky_relu(z, 0.1), bias=b2, x_bound=b, sequential=True)
+
+
 def mlp_leaky(mlp, x):
     """bee_layers.MLP: lin_direct(x) + layers(x) with LeakyReLU(0.1) (archs/diffuser_atoms15.py:98-110)."""
-    L = mlp.layers
-    z, b = linear(L[0], x, want_bound=True)
-    z, b = linear(L[2], F.leaky_relu(z, 0.1), x_bound=b, want_bound=True)
-    return linear(mlp.lin_direct, x) + linear(L[4], F.leaky_relu(z, 0.1), x_bound=b)
+    params = [*_mlp_parameters(mlp), mlp.lin_direct.weight]
+    lead, x = x.shape[:-1], x.reshape(-1, x.shape[-1]).contiguous()
+    fused = (mlp.lin_direct.bias is None and not any(t is None or has_tangent(t) for t in (x, *params))
+             and ops.mlp_leaky_takes(x, params[0:6:2] + params[6:], params[1:6:2]))
+    if fused:
+        return _MlpLeaky.apply(x, *params).reshape(*lead, -1)
+    if mlp.lin_direct.bias is None:
+        return _mlp_leaky_rows(params, x).reshape(*lead, -1)
+    return (_mlp_leaky_rows(params, x) + mlp.lin_direct.bias).reshape(*lead, -1)
 
 
 def radial_encode_painn(r, n, rmax):

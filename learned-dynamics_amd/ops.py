@@ -1224,6 +1224,7 @@ def tensor_linear_wgrad(inds, dy, x, dy_bound=None, x_bound=None, want_bias=Fals
 # ------------------------------------------------- PaiNN layers under differentiation (values, or values and tangents)
 mlp_silu_fwd = _ext.mlp_silu_fwd
 mlp_silu_bwd = _ext.mlp_silu_bwd
+mlp_leaky_takes, mlp_leaky_fwd, mlp_leaky_bwd = _ext.mlp_leaky_takes, _ext.mlp_leaky_fwd, _ext.mlp_leaky_bwd
 painn_edge_encode_fwd = _ext.edge_encode_fwd
 painn_edge_encode_bwd = _ext.edge_encode_bwd
 painn_combine_dual_bwd = _ext.combine_dual_bwd

@@ -176,3 +176,43 @@ def test_mlp_summed_over_segments(ops, rows, dim_in, dim):
         big, size = _layers_and_sum(x.double(), W, b, seg, n_out)
         k = seg[rows // 2]
         assert float((odd[k].double() - big[k]).norm() / size[k]) <= 1.5e-6
+
+
+@pytest.mark.parametrize("rows, dim_in, dim, dim_out", [(256, 64, 64, 32), (257, 96, 96, 160), (700, 256, 512, 256),
+                                                         (5000, 64, 128, 64)])
+def test_leaky_mlp_and_its_adjoint(ops, rows, dim_in, dim, dim_out):
+    """Values, hidden rows and all gradients against float64 (its slopes at the kernel's signs, which may differ from its own only
+    where z is within the rounding of a layer of zero); rows as above, weights' gradients in their 2-norm; a row has the
+    same bits among fewer rows."""
+    g = torch.Generator().manual_seed(rows)
+    W = [(torch.randn(o, k, generator=g) * k ** -0.5).cuda() for o, k in ((dim, dim_in), (dim, dim), (dim_out, dim), (dim_out, dim_in))]
+    b = [(torch.randn(w.shape[0], generator=g) * 0.1).cuda() for w in W[:3]]
+    x, dy = (torch.randn(rows, k, generator=g).cuda() for k in (dim_in, dim_out))
+    assert ops.mlp_leaky_takes(x, W, b)
+    y, saved = ops.mlp_leaky_fwd(x, W, b)
+    Wd, bd, h, slopes, hs = [w.double() for w in W], [t.double() for t in b], x.double(), [], [x.double()]
+    for k in range(2):
+        z = h @ Wd[k].t() + bd[k]
+        kernel = saved[1 + 2 * k]
+        assert not bool((((z > 0) != (kernel > 0)) & (z.abs() > 2e-6 * z.norm(dim=1, keepdim=True))).any())
+        slopes.append(torch.where(kernel > 0, 1.0, 0.1).double())
+        h = z * slopes[-1]
+        hs.append(h)
+        _assert_rows(kernel, h, ("h", k))
+        assert torch.equal(saved[2 + 2 * k][:, 0], kernel.abs().amax(1))
+    assert torch.equal(saved[0][:, 0], x.abs().amax(1))
+    _assert_rows(y, h @ Wd[2].t() + bd[2] + hs[0] @ Wd[3].t(), "y")
+    g_x, params = ops.mlp_leaky_bwd(dy, x, W, saved, True, True)
+    d = dy.double()
+    dz2 = (d @ Wd[2]) * slopes[1]
+    dz1 = (dz2 @ Wd[1]) * slopes[0]
+    _assert_rows(g_x, dz1 @ Wd[0] + d @ Wd[3], "g_x")
+    refs = dz1.t() @ hs[0], dz1.sum(0), dz2.t() @ hs[1], dz2.sum(0), d.t() @ hs[2], d.sum(0), d.t() @ hs[0]
+    for k, (p, r) in enumerate(zip(params, refs)):
+        assert p.shape == r.shape and float((p.double() - r).norm() / r.norm()) <= 1.5e-6, k
+    assert ops.mlp_leaky_bwd(dy, x, W, saved, False, True)[0] is None
+    assert torch.equal(ops.mlp_leaky_fwd(x[:256].contiguous(), W, b)[0], y[:256])
+    x[3, 1] = INF
+    odd, _ = ops.mlp_leaky_fwd(x, W, b)
+    keep = torch.arange(rows, device="cuda") != 3
+    assert torch.equal(odd[keep], y[keep]) and not bool(torch.isfinite(odd[3]).any())
