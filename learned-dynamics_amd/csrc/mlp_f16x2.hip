@@ -218,22 +218,22 @@ __device__ __forceinline__ void split_rows(_Float16* xh, float* row_max, int K, 
 
 // DUAL: the 32 rows of a block are 16 values and their 16 tangents.  LEAKY: LeakyReLU(0.1) in SiLU's place, whose input need not be
 // kept (h has its sign), and a last layer of N columns.
-template <int MI, int NI, int MODE, bool DUAL, bool LEAKY = false>
-__global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const MlpArgs a) {
+template <int MI, int NI, int MODE, bool DUAL, bool LEAKY>
+__device__ __forceinline__ void mlp_rows(const MlpArgs& a, long tile, int widest) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     static_assert(!DUAL || MI == 1, "one block of values and tangents");
     static_assert(!LEAKY || (!DUAL && MODE != kInfer), "LeakyReLU: values under differentiation");
     constexpr bool kTail = MODE == kAdjoint || LEAKY;              // the last layer is not O columns wide
     constexpr int TM = 32 * MI, kRows = DUAL ? 16 : TM;
     constexpr int kSums = MI * NI == 1 ? 2 : 1;                    // (what 128 registers hold)
-    const int O = a.O, widest = a.K > O ? a.K : O;
+    const int O = a.O;
     _Float16* const xh = reinterpret_cast<_Float16*>(lds);
     float* const row_max = reinterpret_cast<float*>(lds + (size_t)TM * widest * 4);      // [waves][TM]
     float* const fixed = row_max + kMaxWaves / NI * TM;                                  // [kMaxDim]
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
     const int m = lane & 31, G = lane >> 5;
-    const long r0 = (long)blockIdx.x * kRows;
+    const long r0 = tile * kRows;
     const bool tangent = DUAL && m >= 16;
     // rows past the end repeat the last one and are not written
     auto row_of = [&](int mi, int mm) {
@@ -472,6 +472,23 @@ __global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const
     }
 }
 
+template <int MI, int NI, int MODE, bool DUAL, bool LEAKY = false>
+__global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const MlpArgs a) {
+    mlp_rows<MI, NI, MODE, DUAL, LEAKY>(a, blockIdx.x, a.K > a.O ? a.K : a.O);
+}
+
+// Two MLPs whose layers are equally wide in one launch: the first `tiles` workgroups are the first one's
+struct MlpPair {
+    MlpArgs job[2];
+    unsigned tiles;
+    int widest;
+};
+template <int MI>
+__global__ void __launch_bounds__(64 * kMaxWaves, 4) mlp_pair_f16x2_kernel(const MlpPair p) {
+    const bool second = blockIdx.x >= p.tiles;
+    mlp_rows<MI, 1, kInfer, false, false>(p.job[second], blockIdx.x - (second ? p.tiles : 0), p.widest);
+}
+
 // Linear, LeakyReLU(0.1), Linear, LeakyReLU(0.1), then the sum over the rows of each segment (seg ascending); the hidden rows stay in
 // LDS and the second layer's in registers.  64 rows a workgroup, wave w owns 32 columns of both layers.  In the second
 // layer the rows are the A operand: a lane holds rows of ONE column, and after a swap of the halves of the wave lanes 0 .. 31
@@ -676,6 +693,20 @@ int choose(const MlpArgs& a, bool dual, hipStream_t st) {
     }
 }
 
+template <int MI>
+int launch_pair(MlpPair& p, hipStream_t st) {
+    p.widest = p.job[0].O;
+    for (const MlpArgs& a : p.job) p.widest = a.K > p.widest ? a.K : p.widest;
+    const size_t lds = (size_t)32 * MI * p.widest * 4 + (kMaxWaves * 32 * MI + kMaxDim) * sizeof(float);
+    if (lds > 65536)
+        MG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mlp_pair_f16x2_kernel<MI>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const long first = ceil_div(p.job[0].R, 32 * MI), tiles = first + ceil_div(p.job[1].R, 32 * MI);
+    MG_REQUIRE(tiles <= 0x7fffffffL, "mg_mlp_f16x2_pair: grid too large");
+    p.tiles = (unsigned)first;
+    hipLaunchKernelGGL(mlp_pair_f16x2_kernel<MI>, dim3((unsigned)tiles), dim3(2 * p.job[0].O), lds, st, p);
+    return check_launch("mg_mlp_f16x2_pair");
+}
+
 // Two column blocks to a wave, so that two workgroups share a CU, where the width has them: by the width alone and not by the rows as
 // above, since the slope at zero should not depend on how many rows a call has.  127 000 rows, 256 -> 512 -> 512 -> 256: 0.57 ms, the
 // adjoint 0.72 (weights out of the L2 at 14 TB/s, 1.3 GB of kept rows); four linears, the activations, their derivatives and the row
@@ -735,6 +766,35 @@ int mg_mlp_f16x2_forward(const mg_mlp_f16x2* p, mg_stream_t stream) {
                    (keep || !p->dual),
                "mg_mlp_f16x2_forward: null or unaligned pointer");
     return keep ? choose<kTrain>(a, p->dual, (hipStream_t)stream) : choose<kInfer>(a, false, (hipStream_t)stream);
+}
+
+int mg_mlp_f16x2_forward_pair(const mg_mlp_f16x2* first, const mg_mlp_f16x2* second, mg_stream_t stream) {
+    MG_REQUIRE(first && second && first->dim == second->dim, "mg_mlp_f16x2_forward_pair: two MLPs of one width");
+    MlpPair p{};
+    const mg_mlp_f16x2* in[2] = {first, second};
+    long tiles = 0;
+    for (int k = 0; k < 2; k++) {
+        const mg_mlp_f16x2& m = *in[k];
+        MlpArgs& a = p.job[k];
+        MG_REQUIRE(m.rows >= 0 && mg_mlp_f16x2_supported(m.dim_in, m.dim) && !m.dual && !m.z[0] && !m.h[0] && !m.x_rowmax,
+                   "mg_mlp_f16x2_forward_pair: inference only, dimensions multiples of 32 up to %d", kMaxDim);
+        a.x = m.x;
+        a.R = m.rows;
+        a.K = m.dim_in;
+        a.O = a.N = m.dim;
+        a.y = m.y;
+        for (int l = 0; l < 3; l++) {
+            a.bias[l] = m.bias[l];
+            MG_REQUIRE(m.packed_W[l] && (!m.bias[l] || aligned16(m.bias[l])), "mg_mlp_f16x2_forward_pair: null or unaligned weight or bias");
+        }
+        MG_REQUIRE(fill(a, m.packed_W, a.K, a.O, a.N) && (m.rows == 0 || (a.x && a.y && aligned16(a.x) && aligned16(a.y))),
+                   "mg_mlp_f16x2_forward_pair: null or unaligned pointer");
+        tiles += ceil_div(m.rows, 32);
+    }
+    if (tiles == 0) return MG_OK;
+    // (the line of one MLP)
+    if (tiles * (first->dim / 32) > 256 * kMaxWaves) return launch_pair<2>(p, (hipStream_t)stream);
+    return launch_pair<1>(p, (hipStream_t)stream);
 }
 
 int mg_mlp_f16x2_adjoint(const mg_mlp_f16x2_grad* p, mg_stream_t stream) {

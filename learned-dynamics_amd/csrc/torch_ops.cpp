@@ -508,13 +508,12 @@ bool mlp_takes(int64_t rows, int64_t k, const Tensors& W, const at::Tensor& x) {
     return aligned16(x);
 }
 
-at::Tensor mlp_fused(const at::Tensor& x, const Tensors& W, const Tensors& b) {
-    at::Tensor y = floats(x, {x.size(0), W[2].size(0)});
+// planes: kept alive by the caller until the launch is queued
+mg_mlp_f16x2 mlp_args(const at::Tensor& x, const Tensors& W, const Tensors& b, at::Tensor& y, Tensors& planes) {
     mg_mlp_f16x2 a{};
-    Tensors planes;                                           // (kept alive until the launch is queued)
     for (int l = 0; l < 3; l++) {
         planes.push_back(packed_f16x2(W[l], l == 0 ? x.size(1) : W[l].size(1)));
-        a.packed_W[l] = planes[l].data_ptr();
+        a.packed_W[l] = planes.back().data_ptr();
         a.bias[l] = fp(b[l]);
     }
     a.x = fp(x);
@@ -522,6 +521,12 @@ at::Tensor mlp_fused(const at::Tensor& x, const Tensors& W, const Tensors& b) {
     a.dim_in = (int)x.size(1);
     a.dim = (int)W[0].size(0);
     a.y = fp(y);
+    return a;
+}
+at::Tensor mlp_fused(const at::Tensor& x, const Tensors& W, const Tensors& b) {
+    at::Tensor y = floats(x, {x.size(0), W[2].size(0)});
+    Tensors planes;
+    const mg_mlp_f16x2 a = mlp_args(x, W, b, y, planes);
     check(mg_mlp_f16x2_forward(&a, stream_of(x)));
     return y;
 }
@@ -647,6 +652,27 @@ at::Tensor filter_grid(const at::Tensor& enc, const at::Tensor& unit, const Tens
     const auto [l1, bmax] = norms_of(W[0], b0);
     check_chain(h, {W[1], W[2]}, {b[1], b[2]}, {kActSilu, kActNone});
     return chain(h, {W[1], W[2]}, {b[1], b[2]}, {kActSilu, kActNone}, Bound{OptTensor(unit), l1, bmax});
+}
+
+// Two of them, in one launch where both go through the MLP kernel
+std::tuple<at::Tensor, at::Tensor> filter_grids(const at::Tensor& enc_0, const at::Tensor& unit_0, const Tensors& W_0, const Tensors& b_0,
+                                                const at::Tensor& enc_1, const at::Tensor& unit_1, const Tensors& W_1, const Tensors& b_1) {
+    auto takes = [&](const at::Tensor& enc, const Tensors& W, const Tensors& b) {
+        return enc.dim() == 2 && enc.size(1) >= W[0].size(1) && mlp_takes(enc.size(0), enc.size(1), W, enc) && aligned_all(b);
+    };
+    if (W_0[0].size(0) != W_1[0].size(0) || enc_0.device() != enc_1.device() || !takes(enc_0, W_0, b_0) || !takes(enc_1, W_1, b_1))
+        return {filter_grid(enc_0, unit_0, W_0, b_0), filter_grid(enc_1, unit_1, W_1, b_1)};
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(enc_0.device());
+    for (const auto& [enc, W, b] : {std::tie(enc_0, W_0, b_0), std::tie(enc_1, W_1, b_1)}) {
+        check_input(enc, "enc");
+        TORCH_CHECK(W.size() == 3 && b.size() == 3, "filter_grids: three layers expected");
+        for (int l = 0; l < 3; l++) check_input(b[l], "bias");
+    }
+    at::Tensor y_0 = floats(enc_0, {enc_0.size(0), W_0[2].size(0)}), y_1 = floats(enc_1, {enc_1.size(0), W_1[2].size(0)});
+    Tensors planes;
+    const mg_mlp_f16x2 a = mlp_args(enc_0, W_0, b_0, y_0, planes), c = mlp_args(enc_1, W_1, b_1, y_1, planes);
+    check(mg_mlp_f16x2_forward_pair(&a, &c, stream_of(enc_0)));
+    return {y_0, y_1};
 }
 
 // Message.forward with the filter interpolated from its grid, which is evaluated here: enc (rows, k) the grid's
@@ -1416,6 +1442,7 @@ void register_ops(pybind11::module_& m) {
     m.def("silu_order", &silu_order);
     m.def("linear_chain", &linear_chain);
     m.def("filter_grid", &filter_grid);
+    m.def("filter_grids", &filter_grids);
     m.def("painn_update", &painn_update);
     m.def("painn_message_grid", &painn_message_grid);
     m.def("painn_message_edges", &painn_message_edges);

@@ -1018,6 +1018,11 @@ def filter_grid(enc, unit, weights, biases):
     return _ext.filter_grid(enc, unit, weights, biases)
 
 
+def filter_grids(first, second):
+    """filter_grid of two sets of arguments, in one launch where their layers have one width."""
+    return _ext.filter_grids(*first, *second)
+
+
 def painn_update(x_a, x_v, W_lrv, weights, biases, gn, residual):
     """Update.forward (archs/meanflow_painn8.py:63-75) in one host call: the stacked l, r, v maps, the MLP, the norm gn and
     the gated vectors.  (out_a, out_v), with residual on top of x_a and x_v."""

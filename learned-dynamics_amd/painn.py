@@ -367,9 +367,18 @@ class Message(nn.Module):
             cache.update(stamp=stamp, trained=training)
         return cache["rows"]
 
-    def forward(self, graph: Graph, x_a, x_v, r_ij, residual=False):
+    def _grid_rows(self, E, n):
+        """(rows, sliced) of the filter grid that a forward pass over E edges reads, or None where it reads none."""
+        if not (self.use_table and isinstance(self.mlp_dist, MLP) and n % 4 == 0 and E >= 4 * self.TABLE_ROWS[0]):
+            return None
+        rows = self.table_rows()
+        sliced = rows and rows <= ops.PAINN_SLICED_MAX_ROWS and n % ops.PAINN_SLICE == 0 and self.use_sliced
+        return (rows, sliced) if sliced or (rows and E >= 4 * rows) else None
+
+    def forward(self, graph: Graph, x_a, x_v, r_ij, residual=False, table=None):
         """x_a: (batch, atoms, n), x_v: (batch, atoms, n, 3), r_ij: (edges, 3).
-        Returns (dx_a, dx_v), or (x_a + dx_a, x_v + dx_v) with residual=True."""
+        Returns (dx_a, dx_v), or (x_a + dx_a, x_v + dx_v) with residual=True.  table: the filter's grid of this call
+        (filter_table of the rows that _grid_rows names), if the caller has it already."""
         if diff.wants_grad(self, x_a, x_v, r_ij):
             da, dv = diff.painn_message(self, graph, x_a, x_v, r_ij)
             return (diff.add(x_a, da), diff.add(x_v, dv)) if residual else (da, dv)
@@ -380,25 +389,25 @@ class Message(nn.Module):
         plain = actv_mlp is not None and dist_mlp is not None
         flat_a, flat_v = x_a.reshape(B * N, n), x_v.reshape(B * N, n, 3)
         res_a, res_v = (flat_a, flat_v) if residual else (None, None)
-        if self.use_table and isinstance(self.mlp_dist, MLP) and n % 4 == 0 and E >= 4 * self.TABLE_ROWS[0]:
-            rows = self.table_rows()
-            sliced = rows and rows <= ops.PAINN_SLICED_MAX_ROWS and n % ops.PAINN_SLICE == 0 and self.use_sliced
-            if (sliced or (rows and E >= 4 * rows)) and not plain:
+        grid = self._grid_rows(E, n)
+        if grid is not None:
+            rows, sliced = grid
+            if not plain:
                 # (the submodules called as such: hooks, something else in their place)
                 out_a, out_v = ops.painn_table_message(graph.row_ptr, graph.dst32, r_ij, self.filter_table(rows), 2.0 * self.r0,
                                                        self.mlp_actv(flat_a), flat_v, self.epsilon, res_a, res_v)
                 return out_a.reshape(B, N, n), out_v.reshape(B, N, n, 3)
-            if sliced or (rows and E >= 4 * rows):
-                # The grid is re-evaluated in every call (a few thousand rows): nothing of a forward is cached.  Where it
-                # fits in LDS, actv comes out of its MLP with the columns regrouped slice by slice, and the rows are taken
-                # in cell order when the graph has one: consecutive rows then gather the same neighbours.
-                order = getattr(graph, "cell_order", None) if sliced and self.use_cell_order else None
-                table = self.filter_table(rows) if self.keep_table else None
-                if sliced:
-                    last, (W, b) = self._sliced_actv_last(), actv_mlp
-                    actv_mlp = [*W[:2], last.weight], [*b[:2], last.bias]
-                return ops.painn_message_grid(graph.row_ptr, graph.dst32, r_ij, order, x_a, x_v, *actv_mlp,
-                                              *self._grid_inputs(dist_mlp, rows), table, 2.0 * self.r0, self.epsilon, sliced, residual)
+            # The grid is re-evaluated in every call (a few thousand rows): nothing of a forward is cached.  Where it
+            # fits in LDS, actv comes out of its MLP with the columns regrouped slice by slice, and the rows are taken
+            # in cell order when the graph has one: consecutive rows then gather the same neighbours.
+            order = getattr(graph, "cell_order", None) if sliced and self.use_cell_order else None
+            if self.keep_table:
+                table = self.filter_table(rows)
+            if sliced:
+                last, (W, b) = self._sliced_actv_last(), actv_mlp
+                actv_mlp = [*W[:2], last.weight], [*b[:2], last.bias]
+            return ops.painn_message_grid(graph.row_ptr, graph.dst32, r_ij, order, x_a, x_v, *actv_mlp,
+                                          *self._grid_inputs(dist_mlp, rows), table, 2.0 * self.r0, self.epsilon, sliced, residual)
         if getattr(graph, "padded", False):
             # the edge arrays are longer than the graph: only the kernels above, which reach the edges through
             # row_ptr, are valid; the per-edge GEMMs below would also process the rows past the edge count
@@ -442,13 +451,32 @@ class Block(nn.Module):
         if self.pos_mutable:
             self.lin_push_pos = TensLinear(1, n, 1)
 
+    def _filter_grids(self, x_a, x_v, r_ij_bond, r_ij):
+        """The two messages' filter grids as their keyword arguments, evaluated together: a grid does not depend on the
+        features, and one of 4096 rows occupies half the chip (128 workgroups; two in a launch 50 us, one after the other 87).
+        Empty where a message makes its own: recorded for differentiation, without a grid or with one it keeps, or called with
+        hooks, which see its arguments."""
+        messages = (self.message_bond, self.message)
+        if diff.wants_grad(self, x_a, x_v, r_ij_bond, r_ij) or not all(diff.plain_call(m, Message) for m in messages):
+            return {}, {}
+        inputs = []
+        for m, r in zip(messages, (r_ij_bond, r_ij)):
+            params = None if m.keep_table or _plain_params(m.mlp_actv) is None else _plain_params(m.mlp_dist)
+            grid = m._grid_rows(r.shape[0], x_a.shape[2]) if params is not None else None
+            if grid is None:
+                return {}, {}
+            inputs.append(m._grid_inputs(params, grid[0]))
+        return tuple({"table": t} for t in ops.filter_grids(*inputs))
+
     def forward(self, tup):
         pos, graph, r_ij, graph_bond, r_ij_bond, x_a, x_v, box = tup
         if graph is None:
             graph, r_ij = graph_setup(self.r0, box, pos)
+        bond = pair = {}
         if graph_bond is not None:
-            x_a, x_v = self.message_bond(graph_bond, x_a, x_v, r_ij_bond, residual=True)
-        x_a, x_v = self.message(graph, x_a, x_v, r_ij, residual=True)
+            bond, pair = self._filter_grids(x_a, x_v, r_ij_bond, r_ij)
+            x_a, x_v = self.message_bond(graph_bond, x_a, x_v, r_ij_bond, residual=True, **bond)
+        x_a, x_v = self.message(graph, x_a, x_v, r_ij, residual=True, **pair)
         x_a, x_v = self.update(x_a, x_v, residual=True)
         if self.pos_mutable:
             pos = diff.add(pos, self.lin_push_pos(x_v).squeeze(-2))

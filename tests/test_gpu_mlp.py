@@ -216,3 +216,25 @@ def test_leaky_mlp_and_its_adjoint(ops, rows, dim_in, dim, dim_out):
     odd, _ = ops.mlp_leaky_fwd(x, W, b)
     keep = torch.arange(rows, device="cuda") != 3
     assert torch.equal(odd[keep], y[keep]) and not bool(torch.isfinite(odd[3]).any())
+
+
+@pytest.mark.parametrize("rows, dim_in, dim", [((1, 33), (64, 96), 64), ((512, 4096), (64, 64), 512), ((4096, 700), (64, 160), 256),
+                                               ((9000, 8000), (64, 128), 512)])
+def test_two_mlps_in_one_launch(ops, rows, dim_in, dim):
+    """The grids of two filters of one width together, on either side of the line to 64 rows a workgroup."""
+    unit = torch.ones(1, 1).cuda()
+    jobs = []
+    for k in range(2):
+        W, b = _weights(dim_in[k], dim, seed=k)
+        x = torch.rand(rows[k], dim_in[k], generator=torch.Generator().manual_seed(k)).cuda() * 2 - 1
+        jobs.append((x, unit, W, b))
+    for y, (x, _, W, b) in zip(ops.filter_grids(*jobs), jobs):
+        _assert_rows(y, _formula(x.double(), W, b), (rows, dim_in, dim))
+    # layers of two widths, and encodings that end in zero columns
+    (x, _, W, b), other = jobs[0], _weights(64, 96)
+    alone = ops.filter_grid(x, unit, W, b), ops.filter_grid(x[:, :64].contiguous(), unit, *other)
+    assert all(torch.equal(p, q) for p, q in zip(ops.filter_grids((x, unit, W, b), (x[:, :64].contiguous(), unit, *other)), alone))
+    narrow = [W[0][:, :48].contiguous(), *W[1:]]
+    padded = torch.cat([x[:, :48], torch.zeros_like(x[:, 48:])], dim=1)
+    for y in ops.filter_grids((padded, unit, narrow, b), (padded, unit, narrow, b)):
+        _assert_rows(y, _formula(x[:, :48].double(), narrow, b), "zero columns")

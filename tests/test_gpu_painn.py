@@ -680,3 +680,24 @@ def test_message_with_the_grid_in_lds_over_nodes_of_any_degree(pkg, degrees, ord
         want_a, want_b = ops.painn_table_message(row_ptr, dst, r, table, period, actv, v, 0.1, *res)
         for x, y in ((a, want_a), (b, want_b)):
             assert float((x - y).abs().max()) <= 2 ** -24 * (8 * max(1, max(degrees)) ** 0.5 + rows) * max(1.0, float(y.abs().max()))
+
+
+@pytest.mark.parametrize("E_bond, n", [(9000, 64), (300, 64), (20000, 128)])
+def test_block_with_both_filter_grids_in_one_launch(pkg, E_bond, n):
+    """A block of two graphs against its messages called one by one (a hook that changes nothing keeps a block from handing
+    a message its grid), where both, or only the second, read a grid: the same kernels on the same rows, bit for bit."""
+    painn = importlib.import_module("learned-dynamics_amd.painn")
+    gl = importlib.import_module("learned-dynamics_amd.graph_layers")
+    torch.manual_seed(0x947 + n)
+    N = 120
+    edges = []
+    for E in (E_bond, 12000):
+        src, dst = torch.sort(torch.randint(0, N, (E,))).values, torch.randint(0, N, (E,))
+        edges += [gl.Graph(src.cuda(), dst.cuda(), None, 1, N), torch.randn(E, 3).cuda()]
+    x_a, x_v = torch.randn(1, N, n).cuda(), torch.randn(1, N, n, 3).cuda()
+    block = painn.Block(5.0, n, n_rbf=16).cuda().requires_grad_(False)
+    got = block((None, edges[2], edges[3], edges[0], edges[1], x_a, x_v, None))
+    hook = block.message.register_forward_hook(lambda *a: None)
+    want = block((None, edges[2], edges[3], edges[0], edges[1], x_a, x_v, None))
+    hook.remove()
+    assert torch.equal(got[5], want[5]) and torch.equal(got[6], want[6])
