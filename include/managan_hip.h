@@ -853,6 +853,12 @@ int mg_tensor_linear_f16x2_rowsum_scaled_bound(const void* packed_W, const float
                                                const int* seg, long n_out, float scale, void* workspace, float* y,
                                                float* out, float bound_mul, float bound_add, mg_stream_t stream);
 
+/* The maps lin_l, lin_r, lin_v of Update.forward (archs/meanflow_painn8.py:63-75) and mg_painn_update_pre in one: x_v (rows, n, 3), x_a
+ * (rows, n), packed_W the packed weight of the three maps below one another, (3n, n) -> ip, cat and cat_rowmax as there, v (rows, 3, n) =
+ * lin_v(x_v).  mg_painn_update_maps_supported: n a multiple of 32 from 64 to 256.  All pointers but cat_rowmax 16-byte aligned. */
+int mg_painn_update_maps_supported(int n);      /* returns 0 / 1, not a status */
+int mg_painn_update_maps(const float* x_v, const float* x_a, long rows, int n, const void* packed_W, float* ip, float* cat,
+                         float* cat_rowmax, float* v, mg_stream_t stream);
 /* Update.forward (archs/meanflow_painn8.py:63-75), elementwise parts around its GEMMs.
  * lrv = [lin_l | lin_r | lin_v] applied to x_v (one stacked tensor_linear), stored (rows, 3n, 3) as the reference
  * stores tensors (lrv_comp_major = 0) or component-major (rows, 3, 3n) (lrv_comp_major = 1).
@@ -861,6 +867,7 @@ int mg_tensor_linear_f16x2_rowsum_scaled_bound(const void* packed_W, const float
  * The scalar output is mg_group_norm(mode 1) of ip * y[:, n:2n] plus y[:, 2n:3n]. */
 int mg_painn_update_pre(const float* lrv, int lrv_comp_major, const float* x_a, long rows, int n, float* ip, float* cat,
                         float* cat_rowmax /* (rows) max |cat[r,:]|, or NULL; n <= 256 */, mg_stream_t stream);
+/* (lrv_comp_major = 2: lrv is lin_v(x_v) alone, (rows, 3, n)) */
 int mg_painn_update_vec(const float* lrv, int lrv_comp_major, const float* y, const float* res_v /* or NULL */, long rows, int n,
                         float* out_v, mg_stream_t stream);
 

@@ -100,6 +100,8 @@ _SIGNATURES = {
     "mg_group_norm_scratch_bytes": [i32, i32, ctypes.POINTER(ctypes.c_size_t)],
     "mg_group_norm": [i32, vp, i64, vp, i64, i32, i32, i32, i32, i32, f32, vp, vp, vp, i64, vp, vp, vp, vp],
     "mg_tens_sigmoid": [i32, vp, i64, vp, vp],
+    "mg_painn_update_maps_supported": [i32],
+    "mg_painn_update_maps": [vp, vp, i64, i32, vp, vp, vp, vp, vp, vp],
     "mg_painn_update_pre": [vp, i32, vp, i64, i32, vp, vp, vp, vp],
     "mg_painn_update_vec": [vp, i32, vp, vp, i64, i32, vp, vp],
     "mg_radial_encode": [i32, vp, i64, i32, f32, vp, vp],

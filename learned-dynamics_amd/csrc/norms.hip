@@ -184,18 +184,18 @@ __global__ void __launch_bounds__(256) painn_update_pre_kernel(const float* __re
     }
 }
 
-// PaiNN Update, vector output: v = lin_v(x_v) * y[0:n]; out = res_v + v / sqrt(1 + |v|^2), out (rows, n, 3)
-template <bool COMP_MAJOR>
+// PaiNN Update, vector output: v = lin_v(x_v) * y[0:n]; out = res_v + v / sqrt(1 + |v|^2), out (rows, n, 3).  LAYOUT: of lrv, as
+// lrv_comp_major of mg_painn_update_vec
+template <int LAYOUT>
 __global__ void __launch_bounds__(256) painn_update_vec_kernel(const float* __restrict__ lrv, const float* __restrict__ y,
                                                                const float* __restrict__ res_v, int n,
                                                                float* __restrict__ out_v) {
     const long r = blockIdx.x;
     const int c = blockIdx.y * blockDim.x + threadIdx.x;
     if (c >= n) return;
-    const float* row = lrv + r * 9 * n;
     const float s = y[r * 3 * n + c];
-    const float a = lrv_at<COMP_MAJOR>(row, n, 2 * n + c, 0) * s, b = lrv_at<COMP_MAJOR>(row, n, 2 * n + c, 1) * s,
-                d = lrv_at<COMP_MAJOR>(row, n, 2 * n + c, 2) * s;
+    auto v_at = [&](int x) { return LAYOUT == 2 ? lrv[(r * 3 + x) * n + c] : lrv_at<LAYOUT == 1>(lrv + r * 9 * n, n, 2 * n + c, x); };
+    const float a = v_at(0) * s, b = v_at(1) * s, d = v_at(2) * s;
     const float inv = 1.0f / sqrtf(1.0f + (a * a + b * b + d * d));
     float o0 = a * inv, o1 = b * inv, o2 = d * inv;
     const long t = r * n + c;
@@ -307,10 +307,8 @@ int mg_painn_update_vec(const float* lrv, int lrv_comp_major, const float* y, co
     MG_REQUIRE(rows <= 0x7fffffffL, "mg_painn_update_vec: more than 2^31 - 1 rows");
     const int threads = n >= 256 ? 256 : (int)ceil_div(n, kWave) * kWave;
     const dim3 grid((unsigned)rows, (unsigned)ceil_div(n, threads));
-    if (lrv_comp_major)
-        hipLaunchKernelGGL(painn_update_vec_kernel<true>, grid, dim3(threads), 0, (hipStream_t)stream, lrv, y, res_v, n, out_v);
-    else
-        hipLaunchKernelGGL(painn_update_vec_kernel<false>, grid, dim3(threads), 0, (hipStream_t)stream, lrv, y, res_v, n, out_v);
+    const auto kernel = lrv_comp_major == 2 ? painn_update_vec_kernel<2> : (lrv_comp_major ? painn_update_vec_kernel<1> : painn_update_vec_kernel<0>);
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, (hipStream_t)stream, lrv, y, res_v, n, out_v);
     return check_launch("mg_painn_update_vec");
 }
 

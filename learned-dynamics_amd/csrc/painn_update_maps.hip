@@ -1,0 +1,210 @@
+// The three maps l, r, v of PaiNN's Update (archs/meanflow_painn8.py:63-75) and what is made of the first two, in one kernel, in the
+// split-fp16 arithmetic of f16x2.hpp: ip = l . r and |r| per channel, [x_a | |r|] with its row maxima, and v.
+//
+// A workgroup takes the 96 (node, component) rows of 32 nodes, one block of 32 rows a component, so that in the product (weight as
+// the A operand) a lane holds all three components of the same channels of one node: the sums over components need no exchange,
+// and l and r, two thirds of the maps' output, are not stored.  Wave w owns channels [32 w, + 32) of the three maps, l and r
+// together and then v: 96 sums in two sets of accumulators (the small products apart) within 256 registers.
+// Bound by memory in part (16 336 nodes of 128 channels: 83 MB, 18 us) and by what a workgroup does in turn: loads, split, products,
+// stores.  Transposition to rows, a linear with component rows and a pass over (rows, 3, 3n) / this kernel, us: 128 channels 1280
+// nodes 17.2 / 14.9, 5120 31 / 18, 16 336 65 / 30, 40 000 147 / 71; 64 channels 12.0 / 12.1, 21 / 13, 39 / 19, 73 / 37; 256 channels
+// 29 / 30, 51 / 39, 143 / 85, 343 / 222.  Of fewer nodes a kernel of ten workgroups takes longer than three launches (320 nodes
+// 9 .. 16 / 12 .. 28): the caller's line is at 1280.
+#include "common.hpp"
+#include "rows_in_lds.hpp"
+
+namespace mg {
+namespace {
+
+constexpr int kNodes = 32, kMaxN = 256;
+
+struct UpdateMaps {
+    const float *x_v, *x_a;
+    long rows;
+    int n;
+    const _Float16* planes;        // of the three maps below one another, (3n, n)
+    const float* inv;
+    float *ip, *cat, *cat_max, *v;
+};
+
+__global__ void __launch_bounds__(64 * kMaxN / 32, 2) painn_update_maps_kernel(const UpdateMaps a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int n = a.n, x_lo = 3 * kNodes * n, waves = n / 32;
+    _Float16* const xh = reinterpret_cast<_Float16*>(lds);
+    float* const row_max = reinterpret_cast<float*>(lds + (size_t)3 * kNodes * n * 4);   // [3][32]
+    float* const top = row_max + 3 * kNodes;                                              // [1 + waves][32], of x_a and |r|
+    float* const fixed = top + (1 + kMaxN / 32) * kNodes;                                 // [3 n]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m = lane & 31, G = lane >> 5;
+    const long r0 = (long)blockIdx.x * kNodes;
+    const bool marked = has_marks(a.inv, 3 * n, lane);
+    // rows past the end repeat the last one and are not written
+    auto row_of = [&](int mm) { return r0 + mm < a.rows ? r0 + mm : a.rows - 1; };
+
+    for (int grp = wave; grp < kNodes / 8; grp += waves) {         // eight lanes to a node, four channels at a time
+        const int mm = grp * 8 + (lane >> 3), p = lane & 7;
+        const long row = row_of(mm);
+        const bool live = r0 + mm < a.rows;
+        float f[kMaxN / 32][12], mx[3] = {0.f, 0.f, 0.f}, ma = 0.f;
+#pragma unroll
+        for (int j = 0; j < kMaxN / 32; j++)
+            if (32 * j < n) {
+                const float4* src = reinterpret_cast<const float4*>(a.x_v + (row * n + 32 * j + 4 * p) * 3);
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+                    const float4 t = src[k];
+                    f[j][4 * k] = t.x; f[j][4 * k + 1] = t.y; f[j][4 * k + 2] = t.z; f[j][4 * k + 3] = t.w;
+                }
+            }
+#pragma unroll
+        for (int j = 0; j < kMaxN / 32; j++)
+            if (32 * j < n) {
+                const float4 t = *reinterpret_cast<const float4*>(a.x_a + row * n + 32 * j + 4 * p);
+                if (live) *reinterpret_cast<float4*>(a.cat + row * 2 * n + 32 * j + 4 * p) = t;
+                ma = fmaxf(fmaxf(fmaxf(ma, fabsf(t.x)), fabsf(t.y)), fmaxf(fabsf(t.z), fabsf(t.w)));
+#pragma unroll
+                for (int k = 0; k < 12; k++) mx[k % 3] = fmaxf(mx[k % 3], fabsf(f[j][k]));
+            }
+#pragma unroll
+        for (int d = 1; d < 8; d <<= 1) {
+            ma = fmaxf(ma, __shfl_xor(ma, d));
+#pragma unroll
+            for (int x = 0; x < 3; x++) mx[x] = fmaxf(mx[x], __shfl_xor(mx[x], d));
+        }
+        if (p == 0) top[mm] = ma;
+#pragma unroll
+        for (int x = 0; x < 3; x++) {
+            float inv;
+            const float scale = pow2_scale(mx[x], &inv);
+            const bool bits = marked || beyond_split(mx[x]);
+#pragma unroll
+            for (int j = 0; j < kMaxN / 32; j++)
+                if (32 * j < n) {
+                    const float v[4] = {f[j][x], f[j][3 + x], f[j][6 + x], f[j][9 + x]};
+                    const int at = x * kNodes * n + piece_at(mm, 32 * j + 4 * p);
+                    if (bits) store_bits(xh, x_lo, at, v);
+                    else store_pieces(xh, x_lo, at, v, scale);
+                }
+            if (p == 0) row_max[x * kNodes + mm] = mx[x];
+        }
+    }
+    __syncthreads();
+    float isx[3];
+    bool odd[3], any_odd = false;
+#pragma unroll
+    for (int x = 0; x < 3; x++) {
+        const float mx = row_max[x * kNodes + m];
+        pow2_scale(mx, &isx[x]);
+        odd[x] = marked || beyond_split(mx);
+        any_odd |= __any(odd[x]);
+    }
+    const long w_lo = (long)pad256(3 * n) * n;
+    const long row = row_of(m);
+    const bool live = r0 + m < a.rows;
+    const _Float16* w = a.planes + (long)wave * (n >> 5) * 1024;
+    // rows that the pieces cannot carry (all waves see the same ones): their sums for maps [first, first + NI)
+    auto finish = [&](auto& acc, int first) {
+        constexpr int NI = sizeof(acc[0]) / sizeof(floatx16);
+#pragma unroll
+        for (int x = 0; x < 3; x++) {
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    const float4 w4 = *reinterpret_cast<const float4*>(a.inv + (first + ni) * n + 32 * wave + 8 * t + 4 * G);
+                    const float iw[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc[x][ni][4 * t + i] = acc[x][ni][4 * t + i] * isx[x] * iw[i];
+                }
+            if (!any_odd) continue;
+            unsigned rows = (unsigned)__ballot(odd[x]);
+            while (rows) {
+                const int r = __builtin_ctz(rows);
+                rows &= rows - 1;
+                for (int c = tid; c < NI * n; c += blockDim.x)
+                    fixed[c] = lds_row_in_fp32(xh + x * kNodes * n, x_lo, r, a.planes, w_lo, first * n + c, n, a.inv[first * n + c]);
+                __syncthreads();
+#pragma unroll
+                for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+                    for (int q = 0; q < 16; q++) {
+                        const float f = fixed[ni * n + 32 * wave + 8 * (q / 4) + 4 * G + q % 4];
+                        if (m == r) acc[x][ni][q] = f;
+                    }
+                __syncthreads();
+            }
+        }
+    };
+    {
+        floatx16 acc[3][2];
+        multiply<3, 2, 1>(w, w_lo, n, xh, kNodes * n, x_lo, lane, acc, waves);
+        finish(acc, 0);
+        float mr = 0.f;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const int c = 32 * wave + 8 * t + 4 * G;
+            float ip[4], nr[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int q = 4 * t + i;
+                const float x = acc[0][1][q], y = acc[1][1][q], z = acc[2][1][q];
+                ip[i] = acc[0][0][q] * x + acc[1][0][q] * y + acc[2][0][q] * z;
+                nr[i] = sqrtf(x * x + y * y + z * z);
+                mr = fmaxf(mr, nr[i]);
+            }
+            if (live) {
+                *reinterpret_cast<float4*>(a.ip + row * n + c) = make_float4(ip[0], ip[1], ip[2], ip[3]);
+                *reinterpret_cast<float4*>(a.cat + row * 2 * n + n + c) = make_float4(nr[0], nr[1], nr[2], nr[3]);
+            }
+        }
+        mr = fmaxf(mr, __shfl_xor(mr, 32));
+        if (G == 0) top[(1 + wave) * kNodes + m] = mr;
+    }
+    {
+        floatx16 acc[3][1];
+        multiply<3, 1, 1>(w + 2L * waves * (n >> 5) * 1024, w_lo, n, xh, kNodes * n, x_lo, lane, acc);
+        finish(acc, 2);
+        if (live)
+#pragma unroll
+            for (int x = 0; x < 3; x++)
+#pragma unroll
+                for (int t = 0; t < 4; t++)
+                    *reinterpret_cast<float4*>(a.v + (row * 3 + x) * n + 32 * wave + 8 * t + 4 * G) =
+                        make_float4(acc[x][0][4 * t], acc[x][0][4 * t + 1], acc[x][0][4 * t + 2], acc[x][0][4 * t + 3]);
+    }
+    __syncthreads();
+    if (tid < kNodes && r0 + tid < a.rows) {
+        float mx = top[tid];
+        for (int k = 1; k <= waves; k++) mx = fmaxf(mx, top[k * kNodes + tid]);
+        a.cat_max[r0 + tid] = mx;
+    }
+}
+
+}  // namespace
+}  // namespace mg
+
+using namespace mg;
+
+extern "C" {
+
+int mg_painn_update_maps_supported(int n) { return n >= 64 && n <= kMaxN && n % 32 == 0; }
+
+int mg_painn_update_maps(const float* x_v, const float* x_a, long rows, int n, const void* packed_W, float* ip, float* cat,
+                         float* cat_rowmax, float* v, mg_stream_t stream) {
+    MG_REQUIRE(rows >= 0 && mg_painn_update_maps_supported(n), "mg_painn_update_maps: n must be a multiple of 32 from 64 to %d", kMaxN);
+    if (rows == 0) return MG_OK;
+    MG_REQUIRE(x_v && x_a && packed_W && ip && cat && cat_rowmax && v && aligned16(x_v) && aligned16(x_a) && aligned16(packed_W) &&
+                   aligned16(ip) && aligned16(cat) && aligned16(v),
+               "mg_painn_update_maps: null or unaligned pointer");
+    const long tiles = ceil_div(rows, kNodes);
+    MG_REQUIRE(tiles <= 0x7fffffffL, "mg_painn_update_maps: too many rows");
+    UpdateMaps a{x_v, x_a, rows, n, static_cast<const _Float16*>(packed_W), nullptr, ip, cat, cat_rowmax, v};
+    a.inv = reinterpret_cast<const float*>(a.planes + 2L * ((3 * n + 255) / 256 * 256) * n);
+    const size_t lds = (size_t)3 * kNodes * n * 4 + ((3 + 1 + kMaxN / 32) * kNodes + 3 * kMaxN) * sizeof(float);
+    if (lds > 65536)
+        MG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(painn_update_maps_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(painn_update_maps_kernel, dim3((unsigned)tiles), dim3(2 * n), lds, (hipStream_t)stream, a);
+    return check_launch("mg_painn_update_maps");
+}
+
+}  // extern "C"

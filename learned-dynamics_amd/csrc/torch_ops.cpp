@@ -499,6 +499,8 @@ bool aligned_all(const Tensors& t) { return std::all_of(t.begin(), t.end(), [](c
 // at 16 384; 128 -> 128 9.9 / 14.2 at 64).  Distance from float64 at 128 -> 512: 2.3e-7 against 2.2..2.5e-7 with split
 // reductions, 2.75e-7 against 4.1e-7 at 16 336 rows.
 constexpr int64_t kMlpWide = 256, kMlpWideRows = 1024;
+bool packs_f16x2(const at::Tensor& W) { return W.size(1) % 32 == 0 && W.size(1) >= 64 && W.size(0) >= 8; }
+
 bool mlp_takes(int64_t rows, int64_t k, const Tensors& W, const at::Tensor& x) {
     const int64_t dim = W[0].size(0);
     if (mg_get_linear_mode() != kModeF16x2 || rows < (dim > kMlpWide ? kMlpWideRows : 1) || k < 64 || dim < 64 || !mg_mlp_f16x2_supported((int)k, (int)dim))
@@ -592,14 +594,22 @@ std::tuple<at::Tensor, at::Tensor> painn_update(const at::Tensor& x_a, const at:
     check_input(gamma, "gamma");
     check_input(beta, "beta");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x_a.device());
-    const at::Tensor flat_v = x_v.reshape({rows, n, 3});
-    // component-major (rows, 3, 3n): the GEMM stores whole rows, the two kernels below read with unit stride
-    const at::Tensor lrv = std::get<0>(linear_fwd(1, W_lrv, flat_v, OptTensor(), kActNone, OptTensor(), false, 0, 1, OptTensor(),
-                                                  1, 0, 1, false, OptTensor(), OptTensor(), false));
-    at::Tensor ip = floats(x_a, {rows, n}), cat = floats(x_a, {rows, 2 * n}), cat_max;
+    at::Tensor ip = floats(x_a, {rows, n}), cat = floats(x_a, {rows, 2 * n}), lrv, cat_max;
     if (n <= 256) cat_max = floats(x_a, {rows, 1});
     const mg_stream_t st = stream_of(x_a);
-    check(mg_painn_update_pre(fp(lrv), 1, fp(x_a), rows, (int)n, fp(ip), fp(cat), n <= 256 ? fp(cat_max) : nullptr, st));
+    // the rows and widths whose component linear is the split-fp16 one, from 40 workgroups on (figures at the kernel)
+    const bool maps = mg_get_linear_mode() == kModeF16x2 && rows >= 1280 && packs_f16x2(W_lrv) &&
+                      mg_painn_update_maps_supported((int)n) && aligned16(x_v) && aligned16(x_a);
+    if (maps) {
+        lrv = floats(x_a, {rows, 3, n});
+        const at::Tensor planes = packed_f16x2(W_lrv, n);
+        check(mg_painn_update_maps(fp(x_v), fp(x_a), rows, (int)n, planes.data_ptr(), fp(ip), fp(cat), fp(cat_max), fp(lrv), st));
+    } else {
+        // component-major (rows, 3, 3n): the GEMM stores whole rows, the two kernels below read with unit stride
+        lrv = std::get<0>(linear_fwd(1, W_lrv, x_v.reshape({rows, n, 3}), OptTensor(), kActNone, OptTensor(), false, 0, 1, OptTensor(),
+                                     1, 0, 1, false, OptTensor(), OptTensor(), false));
+        check(mg_painn_update_pre(fp(lrv), 1, fp(x_a), rows, (int)n, fp(ip), fp(cat), n <= 256 ? fp(cat_max) : nullptr, st));
+    }
     check_chain(cat, W, b, kSiluMlp);
     at::Tensor y = chain(cat, W, b, kSiluMlp, Bound{n <= 256 ? OptTensor(cat_max) : OptTensor()});          // (rows, 3n)
     at::Tensor out_a = floats(x_a, x_a.sizes()), out_v = floats(x_v, x_v.sizes());
@@ -608,7 +618,7 @@ std::tuple<at::Tensor, at::Tensor> painn_update(const at::Tensor& x_a, const at:
     at::Tensor scratch = bytes_like(x_a, std::max<size_t>(scratch_bytes, 8));
     check(mg_group_norm(1, fp(ip), n, fp(y) + n, 3 * n, (int)B, (int)N, (int)n, groups, 1, (float)eps, fp(gamma), fp(beta),
                         fp(y) + 2 * n, 3 * n, residual ? fp(x_a) : nullptr, scratch.data_ptr(), fp(out_a), st));
-    check(mg_painn_update_vec(fp(lrv), 1, fp(y), residual ? fp(x_v) : nullptr, rows, (int)n, fp(out_v), st));
+    check(mg_painn_update_vec(fp(lrv), maps ? 2 : 1, fp(y), residual ? fp(x_v) : nullptr, rows, (int)n, fp(out_v), st));
     return {out_a, out_v};
 }
 
@@ -782,8 +792,6 @@ at::Tensor stacked(const at::Tensor& p, const OptTensor& t, int64_t cols) {
         return on_storage(p, 0, {2 * rows, cols});
     return at::cat({p.reshape({rows, cols}), t->reshape({rows, cols})});
 }
-
-bool packs_f16x2(const at::Tensor& W) { return W.size(1) % 32 == 0 && W.size(1) >= 64 && W.size(0) >= 8; }
 
 // Packed planes of several weights that the next kernels read, those that are missing in one launch.  `passing`: weights that
 // do not outlive this pass; their planes are returned and not kept.

@@ -701,3 +701,43 @@ def test_block_with_both_filter_grids_in_one_launch(pkg, E_bond, n):
     want = block((None, edges[2], edges[3], edges[0], edges[1], x_a, x_v, None))
     hook.remove()
     assert torch.equal(got[5], want[5]) and torch.equal(got[6], want[6])
+
+
+@pytest.mark.parametrize("rows, n", [(1280, 64), (1281, 96), (1400, 256), (1311, 128), (1300, 224)])
+def test_update_with_its_maps_in_one_kernel(pkg, rows, n):
+    """The update against its formula in float64, where the three maps, the products over components and the row maxima are one
+    kernel (whole blocks of 32 nodes, part of one, one wave to the channels and several).  Tolerance: sums of n terms, their products and
+    the MLP on them, each rounded to 2^-22 of its row: 1e-6 of the 2-norm of the rows, and the norm's division by a spread near one.
+    Then infinite and very large rows, which no other row notices."""
+    painn = importlib.import_module("learned-dynamics_amd.painn")
+    torch.manual_seed(rows + n)
+    upd = painn.Update(n).cuda().requires_grad_(False)
+    x_a, x_v = torch.randn(1, rows, n).cuda(), torch.randn(1, rows, n, 3).cuda()
+
+    def formula(dt, x_a, x_v):
+        p = lambda t: t.detach().to(dt)
+        lin = lambda layer, x: torch.einsum("oi,...ix->...ox", p(layer.W), x.to(dt))
+        l, r, v = (lin(layer, x_v) for layer in (upd.lin_l, upd.lin_r, upd.lin_v))
+        h = torch.cat([x_a.to(dt), r.norm(dim=-1)], dim=-1)
+        for k in (0, 2, 4):
+            layer = upd.mlp.layers[k]
+            h = h @ p(layer.weight).t() + p(layer.bias)
+            h = torch.nn.functional.silu(h) if k < 4 else h
+        z = ((l * r).sum(-1) * h[..., n:2 * n]).reshape(1, rows, upd.gn.groups, -1)
+        mean = z.mean(dim=(1, 3), keepdim=True)
+        z = (z - mean) / torch.sqrt(((z - mean) ** 2).mean(dim=(1, 3), keepdim=True) + upd.gn.epsilon)
+        a = p(upd.gn.gamma) * z.reshape(1, rows, n) + p(upd.gn.beta) + h[..., 2 * n:]
+        v = v * h[..., :n, None]
+        return a, v / torch.sqrt(1 + (v ** 2).sum(-1, keepdim=True))
+
+    got, ref = upd(x_a, x_v), formula(torch.float64, x_a, x_v)
+    for name, x, y in zip(("a", "v"), got, ref):
+        assert float((x.double() - y).norm() / y.norm()) <= 1e-6, name
+    # per node, the vectors do not go through the norm: a row that no piece can carry stays by itself
+    x_v[0, 5, 3, 1], x_v[0, rows - 1] = float("inf"), x_v[0, rows - 1] * 2.0 ** 100
+    odd = upd(x_a, x_v)[1]
+    keep = torch.ones(rows, dtype=torch.bool, device="cuda")
+    keep[[5, rows - 1]] = False
+    assert torch.equal(odd[0, keep], got[1][0, keep])
+    # (|r|^2 of both rows is beyond 2^128: undefined as from any sum of squares in fp32)
+    assert not bool(torch.isfinite(odd[0, ~keep]).any())
