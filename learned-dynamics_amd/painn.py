@@ -368,12 +368,14 @@ class Message(nn.Module):
         return cache["rows"]
 
     def _grid_rows(self, E, n):
-        """(rows, sliced) of the filter grid that a forward pass over E edges reads, or None where it reads none."""
+        """Rows of the filter grid that a forward pass over E edges reads, or 0 where it reads none."""
         if not (self.use_table and isinstance(self.mlp_dist, MLP) and n % 4 == 0 and E >= 4 * self.TABLE_ROWS[0]):
-            return None
+            return 0
         rows = self.table_rows()
-        sliced = rows and rows <= ops.PAINN_SLICED_MAX_ROWS and n % ops.PAINN_SLICE == 0 and self.use_sliced
-        return (rows, sliced) if sliced or (rows and E >= 4 * rows) else None
+        return rows if self._sliced(rows, n) or E >= 4 * rows else 0
+
+    def _sliced(self, rows, n):
+        return 0 < rows <= ops.PAINN_SLICED_MAX_ROWS and n % ops.PAINN_SLICE == 0 and self.use_sliced
 
     def forward(self, graph: Graph, x_a, x_v, r_ij, residual=False, table=None):
         """x_a: (batch, atoms, n), x_v: (batch, atoms, n, 3), r_ij: (edges, 3).
@@ -385,29 +387,31 @@ class Message(nn.Module):
         B, N, n = x_a.shape
         x_a, x_v, r_ij = x_a.contiguous(), x_v.contiguous(), r_ij.contiguous()
         E = r_ij.shape[0]
-        actv_mlp, dist_mlp = _plain_params(self.mlp_actv), _plain_params(self.mlp_dist)
-        plain = actv_mlp is not None and dist_mlp is not None
+        actv_mlp, dist_mlp = _plain_params(self.mlp_actv), _plain_params(self.mlp_dist) if table is None else None
+        plain = actv_mlp is not None and (dist_mlp is not None or table is not None)
         flat_a, flat_v = x_a.reshape(B * N, n), x_v.reshape(B * N, n, 3)
         res_a, res_v = (flat_a, flat_v) if residual else (None, None)
-        grid = self._grid_rows(E, n)
-        if grid is not None:
-            rows, sliced = grid
+        rows = self._grid_rows(E, n) if table is None else table.shape[0]
+        if rows:
+            sliced = self._sliced(rows, n)
             if not plain:
                 # (the submodules called as such: hooks, something else in their place)
-                out_a, out_v = ops.painn_table_message(graph.row_ptr, graph.dst32, r_ij, self.filter_table(rows), 2.0 * self.r0,
+                table = self.filter_table(rows) if table is None else table
+                out_a, out_v = ops.painn_table_message(graph.row_ptr, graph.dst32, r_ij, table, 2.0 * self.r0,
                                                        self.mlp_actv(flat_a), flat_v, self.epsilon, res_a, res_v)
                 return out_a.reshape(B, N, n), out_v.reshape(B, N, n, 3)
             # The grid is re-evaluated in every call (a few thousand rows): nothing of a forward is cached.  Where it
             # fits in LDS, actv comes out of its MLP with the columns regrouped slice by slice, and the rows are taken
             # in cell order when the graph has one: consecutive rows then gather the same neighbours.
             order = getattr(graph, "cell_order", None) if sliced and self.use_cell_order else None
-            if self.keep_table:
+            if table is None and self.keep_table:
                 table = self.filter_table(rows)
             if sliced:
                 last, (W, b) = self._sliced_actv_last(), actv_mlp
                 actv_mlp = [*W[:2], last.weight], [*b[:2], last.bias]
             return ops.painn_message_grid(graph.row_ptr, graph.dst32, r_ij, order, x_a, x_v, *actv_mlp,
-                                          *self._grid_inputs(dist_mlp, rows), table, 2.0 * self.r0, self.epsilon, sliced, residual)
+                                          *((None, None, [], []) if table is not None else self._grid_inputs(dist_mlp, rows)),
+                                          table, 2.0 * self.r0, self.epsilon, sliced, residual)
         if getattr(graph, "padded", False):
             # the edge arrays are longer than the graph: only the kernels above, which reach the edges through
             # row_ptr, are valid; the per-edge GEMMs below would also process the rows past the edge count
@@ -456,16 +460,17 @@ class Block(nn.Module):
         features, and one of 4096 rows occupies half the chip (128 workgroups; two in a launch 50 us, one after the other 87).
         Empty where a message makes its own: recorded for differentiation, without a grid or with one it keeps, or called with
         hooks, which see its arguments."""
-        messages = (self.message_bond, self.message)
-        if diff.wants_grad(self, x_a, x_v, r_ij_bond, r_ij) or not all(diff.plain_call(m, Message) for m in messages):
+        messages, edges = (self.message_bond, self.message), (r_ij_bond.shape[0], r_ij.shape[0])
+        if (min(edges) < 4 * Message.TABLE_ROWS[0] or not all(diff.plain_call(m, Message) for m in messages)
+                or diff.wants_grad(self, x_a, x_v, r_ij_bond, r_ij)):
             return {}, {}
         inputs = []
-        for m, r in zip(messages, (r_ij_bond, r_ij)):
-            params = None if m.keep_table or _plain_params(m.mlp_actv) is None else _plain_params(m.mlp_dist)
-            grid = m._grid_rows(r.shape[0], x_a.shape[2]) if params is not None else None
-            if grid is None:
+        for m, E in zip(messages, edges):
+            params = None if m.keep_table else _plain_params(m.mlp_dist)
+            rows = m._grid_rows(E, x_a.shape[2]) if params is not None else 0
+            if not rows:
                 return {}, {}
-            inputs.append(m._grid_inputs(params, grid[0]))
+            inputs.append(m._grid_inputs(params, rows))
         return tuple({"table": t} for t in ops.filter_grids(*inputs))
 
     def forward(self, tup):
