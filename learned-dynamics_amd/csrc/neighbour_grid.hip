@@ -17,8 +17,8 @@
 //   scan     degrees -> CSR row_ptr (+ per-box edge counts, statistics)
 //   fill     copies the hit rows to row_ptr[i] (exact-size rows, no atomics per
 //            edge, no geometry); a row with more hits than a hit row holds is
-//            swept again by one wave.  graph_fill_kernel (mg_graph_fill) is scan and fill in one, and writes int64
-//            indices, edge vectors and the cell order as well
+//            swept again by one wave.  graph_fill_kernel (mg_graph_fill; graph_fill_dealt_kernel for short
+//            rows) is scan and fill in one, and writes int64 indices, edge vectors and the cell order as well
 //
 // fp32 recipe (this file is compiled with -ffp-contract=off):
 //   w    = remainderf(x - box/2, box) + box/2                 (IEEE remainder)
