@@ -636,15 +636,15 @@ int mg_bee_edge_filters_bwd(const float* enc, const float* rh, const float* g_v,
                             float* d_enc, float* d_rh, mg_stream_t stream);
 
 /* Gradients of the 13 message products of Messages (archs/diffuser_atoms15.py:238-253; chan a multiple of 64:
- * mg_bee_message_grad_supported) for the operands l_0 (n_rows, chan), l_1 (.., 3, chan), l_2 (.., 9, chan), read at dst[e], and for enc
- * (E, chan) and rh (E, 3), which the edge filters enc, enc rh, enc rh (x) rh are made of.  d_P0 (E, 3, chan), d_S1 (n_src, 3, 5, chan),
- * d_S2 (n_src, 9, 5, chan): the gradients of the results of mg_bee_message, in its order (row_ptr: the CSR of the edges, which are
- * sorted by source).  dst_row_ptr / perm: the edges sorted by destination.  Outputs, in the layout of the operands, are
- * null where not wanted; d_0, d_1, d_2 come together.  Sums run in a fixed order. */
+ * mg_bee_message_grad_supported) for the operands l_0 (n_rows, chan), l_1 (.., 3), l_2 (.., 3, 3), read at dst[e], and for enc
+ * (E, chan) and rh (E, 3), which the edge filters enc, enc rh, enc rh (x) rh are made of.  dy, in the order of mg_bee_fwd:
+ * the products 000, 110, 220 hold E rows, the others n_src rows, the gradient of their sums over the edges of a source node
+ * (row_ptr: the CSR of the edges, which are sorted by source).  dst_row_ptr / perm: the edges sorted by destination.
+ * Outputs are null where not wanted; d_0, d_1, d_2 come together.  Sums run in a fixed order. */
 int mg_bee_message_grad_supported(int chan);   /* returns 0 / 1, not a status */
 int mg_bee_message_grad_workspace_bytes(long E, int chan, int want_left, int want_rh, size_t* bytes);
 typedef struct mg_bee_message_grad {
-    const float *l_0, *l_1, *l_2, *enc, *rh, *d_P0, *d_S1, *d_S2;
+    const float *l_0, *l_1, *l_2, *enc, *rh, *dy[13];
     const int *row_ptr, *dst, *dst_row_ptr, *perm;
     long E;
     int n_src, n_rows, chan;
@@ -652,6 +652,18 @@ typedef struct mg_bee_message_grad {
     float *d_0, *d_1, *d_2, *d_enc, *d_rh;
 } mg_bee_message_grad;
 int mg_bee_message_grad_run(const mg_bee_message_grad* args, mg_stream_t stream);
+
+/* The same with everything component-major: l_0 (n_rows, chan), l_1 (.., 3, chan), l_2 (.., 9, chan) and their gradients likewise, and
+ * d_P0 (E, 3, chan), d_S1 (n_src, 3, 5, chan), d_S2 (n_src, 9, 5, chan) the gradients of the results of mg_bee_message, in its order. */
+typedef struct mg_bee_message_grad_rows {
+    const float *l_0, *l_1, *l_2, *enc, *rh, *d_P0, *d_S1, *d_S2;
+    const int *row_ptr, *dst, *dst_row_ptr, *perm;
+    long E;
+    int n_src, n_rows, chan;
+    void* workspace;
+    float *d_0, *d_1, *d_2, *d_enc, *d_rh;
+} mg_bee_message_grad_rows;
+int mg_bee_message_grad_rows_run(const mg_bee_message_grad_rows* args, mg_stream_t stream);
 
 /* SiLU and its derivatives for the MLPs' training path (nn.SiLU in archs/meanflow_painn8.py:38-51, differentiated up
  * to three times by the meanflow loss, :274-296): out[k] = SiLU^(order)(z[k]) (* mul[k] if mul is not null), order 0..4,

@@ -126,6 +126,7 @@ _SIGNATURES = {
     "mg_bee_message_grad_supported": [i32],
     "mg_bee_message_grad_workspace_bytes": [i64, i32, i32, i32, vp],
     "mg_bee_message_grad_run": [vp, vp],
+    "mg_bee_message_grad_rows_run": [vp, vp],
     "mg_sort_by_key_workspace_bytes": [i64, vp],
     "mg_painn_grid_rows_by_node_workspace_bytes": [i32, vp],
     "mg_painn_grid_rows_by_node": [vp, i64, vp, vp, i32, i32, f32, vp, vp, vp, vp],

@@ -13,10 +13,12 @@
 // node and not twice per edge; no filters are formed in memory.  dl leaves component-major (E, 13, chan), whole 256-byte
 // rows, and a second kernel sums it over the edges of each destination in a fixed order.
 // What bounds it: traffic, 17 floats read and 14 written per edge and channel, then 13 read.  131 000 edges, 8192 nodes, 256
-// channels, edge vectors not differentiated: 0.70 ms (6.0 TB/s) and 0.44 ms (4.1 TB/s).  Operands and gradients are component-major,
-// a wave's accesses 256 bytes each: the results of the forward kernel and of the output linears as they are.  Before, the filters were stored
+// channels, edge vectors not differentiated: 0.70 ms (6.0 TB/s) and 0.44 ms (4.1 TB/s).  Before, the filters were stored
 // (0.44 ms), two kernels gathered the 60 gradients at every edge's source (1.8 ms each), a third took the right operands'
 // gradients to enc and rh (0.35 ms) and three segment sums followed (0.37 ms).
+// Two layouts of operands and gradients: ROWS is component-major, (row, comp, product, chan), the results of the forward kernel
+// and of the output linears as they are, a wave's accesses 256 bytes each; the other has every product by itself, (row, chan, comp),
+// for callers that hold them so (a module whose linears are called one by one): 0.72 and 0.42 ms, nothing to transpose around it.
 // Any multiple of 64 channels; differentiable.message_products comes here for multiples of 256, the widths of its forward
 // kernels, and keeps the plain formulation for others.
 // The per-edge gradients are stored rather than formed again by destination, which would gather the 60 floats of the source
@@ -37,27 +39,34 @@ __device__ __forceinline__ void cross3(const float* a, const float* b, float* o)
     o[1] = a[2] * b[0] - a[0] * b[2];
     o[2] = a[0] * b[1] - a[1] * b[0];
 }
-// T values `stride` apart
-template <int T>
-__device__ __forceinline__ void load(const float* p, long stride, float* o) {
+// the T components of channel c of a row: (row, T, product, chan) of PRODUCTS products side by side, p at the first row's channel 0
+// of the product, or (row, chan, T)
+template <bool ROWS, int T, int PRODUCTS = 1>
+__device__ __forceinline__ void load(const float* p, long row, long C, int c, float* o) {
+    const float* q = ROWS ? p + row * (T * PRODUCTS) * C + c : p + (row * C + c) * T;
+    const long step = ROWS ? PRODUCTS * C : 1;
 #pragma unroll
-    for (int k = 0; k < T; k++) o[k] = p[k * stride];
+    for (int k = 0; k < T; k++) o[k] = q[k * step];
 }
 
+template <bool ROWS>
 __device__ __forceinline__ EdgeIn load_edge(const mg_bee_message_grad& a, long e, int node, int c) {
     EdgeIn in;
     const long C = a.chan;
-    in.l[0] = a.l_0[node * C + c];
-    load<3>(a.l_1 + node * 3 * C + c, C, in.l + 1);
-    load<9>(a.l_2 + node * 9 * C + c, C, in.l + 4);
+    load<ROWS, 1>(a.l_0, node, C, c, in.l);
+    load<ROWS, 3>(a.l_1, node, C, c, in.l + 1);
+    load<ROWS, 9>(a.l_2, node, C, c, in.l + 4);
     in.enc = a.enc[e * C + c];
-    load<3>(a.d_P0 + e * 3 * C + c, C, in.s);
-    load<3>(a.rh + 3 * e, 1, in.u);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        load<ROWS, 1, 3>(a.dy[k], e, C, c, in.s + k);
+        in.u[k] = a.rh[3 * e + k];
+    }
     return in;
 }
 
 // LEFT: the operands' gradients per edge; RIGHT: d_enc; VEC: d_rh, a sum over this wave's 64 channels
-template <bool LEFT, bool RIGHT, bool VEC>
+template <bool ROWS, bool LEFT, bool RIGHT, bool VEC>
 __global__ void __launch_bounds__(256, 3) bee_message_grad_kernel(mg_bee_message_grad a, long items, long blocks_per_xcd,
                                                                   float* __restrict__ dl, float* __restrict__ part) {
     const int lane = threadIdx.x & 63;
@@ -70,27 +79,25 @@ __global__ void __launch_bounds__(256, 3) bee_message_grad_kernel(mg_bee_message
     const long begin = a.row_ptr[node], end = a.row_ptr[node + 1];
     if (begin >= end) return;
     float g011[3], g101[3], g121[3], g211[3], g111[3], g022[9], g202[9], g112[9], g222[9], g212[9];
-    const float *s1 = a.d_S1 + (long)node * 15 * C + c, *s2 = a.d_S2 + (long)node * 45 * C + c;
-    const long step = 5L * C;
-    load<3>(s1, step, g011);
-    load<3>(s1 + C, step, g101);
-    load<3>(s1 + 2 * C, step, g121);
-    load<3>(s1 + 3 * C, step, g211);
-    load<3>(s1 + 4 * C, step, g111);
-    load<9>(s2, step, g022);
-    load<9>(s2 + C, step, g202);
-    load<9>(s2 + 2 * C, step, g112);
-    load<9>(s2 + 3 * C, step, g222);
-    load<9>(s2 + 4 * C, step, g212);
+    load<ROWS, 3, 5>(a.dy[3], node, C, c, g011);
+    load<ROWS, 3, 5>(a.dy[4], node, C, c, g101);
+    load<ROWS, 3, 5>(a.dy[5], node, C, c, g121);
+    load<ROWS, 3, 5>(a.dy[6], node, C, c, g211);
+    load<ROWS, 9, 5>(a.dy[7], node, C, c, g022);
+    load<ROWS, 9, 5>(a.dy[8], node, C, c, g202);
+    load<ROWS, 9, 5>(a.dy[9], node, C, c, g112);
+    load<ROWS, 9, 5>(a.dy[10], node, C, c, g222);
+    load<ROWS, 3, 5>(a.dy[11], node, C, c, g111);
+    load<ROWS, 9, 5>(a.dy[12], node, C, c, g212);
     auto destination = [&](long e) {
         const int d = a.dst[e];
         return d < 0 ? 0 : (d >= a.n_rows ? a.n_rows - 1 : d);
     };
-    EdgeIn next = load_edge(a, begin, destination(begin), c);
+    EdgeIn next = load_edge<ROWS>(a, begin, destination(begin), c);
     for (long e = begin; e < end; e++) {
         const EdgeIn in = next;
         const long f = e + 1 < end ? e + 1 : e;              // (the next edge's operands are under way during this one's sums)
-        next = load_edge(a, f, destination(f), c);
+        next = load_edge<ROWS>(a, f, destination(f), c);
         const float *u = in.u, *l1 = in.l + 1, *l2 = in.l + 4;
         const float s110 = in.s[1], s220 = in.s[2], gu = dot3(g121, u);
         float w[3], h[3], o[kLeft], t[3];
@@ -162,6 +169,7 @@ __global__ void __launch_bounds__(256) bee_message_grad_rh_kernel(const float* _
 
 // (E, 13, chan) rows summed over the edges of each destination, in the order of its sorted edges; one wave per node and 64
 // channels, two edges in flight
+template <bool ROWS>
 __global__ void __launch_bounds__(256) bee_message_grad_sum_kernel(const float* __restrict__ dl, const int* __restrict__ row_ptr,
                                                                    const int* __restrict__ perm, long items, long blocks_per_xcd,
                                                                    int C, float* __restrict__ d_0, float* __restrict__ d_1,
@@ -187,24 +195,56 @@ __global__ void __launch_bounds__(256) bee_message_grad_sum_kernel(const float* 
 #pragma unroll
         for (int j = 0; j < kLeft; j++) s[j] += p[(long)j * C];
     }
-    d_0[(long)node * C + c] = s[0];
+    const long at = (long)node * C + c;
+    d_0[at] = s[0];
 #pragma unroll
-    for (int j = 0; j < 3; j++) d_1[((long)node * 3 + j) * C + c] = s[1 + j];
+    for (int j = 0; j < 3; j++) d_1[ROWS ? ((long)node * 3 + j) * C + c : 3 * at + j] = s[1 + j];
 #pragma unroll
-    for (int j = 0; j < 9; j++) d_2[((long)node * 9 + j) * C + c] = s[4 + j];
+    for (int j = 0; j < 9; j++) d_2[ROWS ? ((long)node * 9 + j) * C + c : 9 * at + j] = s[4 + j];
 }
 
 // floats of the two pieces of the workspace: the operands' gradients per edge, and d_rh's sums per 64 channels
 size_t left_floats(long E, int chan) { return (size_t)E * kLeft * chan; }
 size_t part_floats(long E, int chan) { return ((size_t)E * (chan / 64) * 3 + 3) / 4 * 4; }
 
-template <bool LEFT, bool RIGHT>
+template <bool ROWS, bool LEFT, bool RIGHT>
 void launch(const mg_bee_message_grad& a, bool vec, long items, long per_xcd, float* dl, float* part, hipStream_t st) {
     const dim3 grid((unsigned)(per_xcd * kXcds));
     if (vec)
-        hipLaunchKernelGGL((bee_message_grad_kernel<LEFT, RIGHT, true>), grid, dim3(256), 0, st, a, items, per_xcd, dl, part);
+        hipLaunchKernelGGL((bee_message_grad_kernel<ROWS, LEFT, RIGHT, true>), grid, dim3(256), 0, st, a, items, per_xcd, dl, part);
     else
-        hipLaunchKernelGGL((bee_message_grad_kernel<LEFT, RIGHT, false>), grid, dim3(256), 0, st, a, items, per_xcd, dl, part);
+        hipLaunchKernelGGL((bee_message_grad_kernel<ROWS, LEFT, RIGHT, false>), grid, dim3(256), 0, st, a, items, per_xcd, dl, part);
+}
+
+template <bool ROWS>
+int run(const char* what, const mg_bee_message_grad& a, mg_stream_t stream) {
+    MG_REQUIRE(mg_bee_message_grad_supported(a.chan), "%s: chan = %d is no multiple of 64", what, a.chan);
+    MG_REQUIRE(a.E >= 0 && a.E < (1L << 31) && a.n_src >= 0 && a.n_rows >= 0, "%s: bad size", what);
+    const bool left = a.d_0 || a.d_1 || a.d_2, right = a.d_enc != nullptr, vec = a.d_rh != nullptr;
+    MG_REQUIRE(!left || (a.d_0 && a.d_1 && a.d_2 && a.dst_row_ptr), "%s: the three operands' gradients come together", what);
+    hipStream_t st = (hipStream_t)stream;
+    const long slices = a.chan / 64, items = (long)a.n_src * slices, sums = (long)a.n_rows * slices;
+    MG_REQUIRE(items < (1L << 31) - 64 && sums < (1L << 31) - 64, "%s: too many nodes", what);
+    float *dl = static_cast<float*>(a.workspace), *part = dl + (left ? left_floats(a.E, a.chan) : 0);
+    if (a.E > 0 && (left || right || vec)) {
+        MG_REQUIRE(a.row_ptr && a.dst && a.rh && a.enc && a.l_0 && a.l_1 && a.l_2 && a.n_rows > 0 && (a.workspace || !(left || vec)),
+                   "%s: null pointer", what);
+        for (int k = 0; k < 13; k++) MG_REQUIRE(a.dy[k], "%s: gradient %d is null", what, k);
+        const long per_xcd = ceil_div(ceil_div(items, 4), kXcds);
+        if (left && right) launch<ROWS, true, true>(a, vec, items, per_xcd, dl, part, st);
+        else if (left) launch<ROWS, true, false>(a, vec, items, per_xcd, dl, part, st);
+        else if (right) launch<ROWS, false, true>(a, vec, items, per_xcd, dl, part, st);
+        else launch<ROWS, false, false>(a, vec, items, per_xcd, dl, part, st);
+        if (vec)
+            hipLaunchKernelGGL(bee_message_grad_rh_kernel, dim3((unsigned)ceil_div(3 * a.E, 256)), dim3(256), 0, st, part, 3 * a.E,
+                               (int)slices, a.d_rh);
+    }
+    if (left && sums > 0) {
+        const long per_xcd = ceil_div(ceil_div(sums, 4), kXcds);
+        hipLaunchKernelGGL(bee_message_grad_sum_kernel<ROWS>, dim3((unsigned)(per_xcd * kXcds)), dim3(256), 0, st, dl, a.dst_row_ptr, a.perm,
+                           sums, per_xcd, a.chan, a.d_0, a.d_1, a.d_2);
+    }
+    return check_launch(what);
 }
 
 }  // namespace
@@ -224,33 +264,26 @@ int mg_bee_message_grad_workspace_bytes(long E, int chan, int want_left, int wan
 
 int mg_bee_message_grad_run(const mg_bee_message_grad* args, mg_stream_t stream) {
     MG_REQUIRE(args, "mg_bee_message_grad_run: null pointer");
-    const mg_bee_message_grad& a = *args;
-    MG_REQUIRE(mg_bee_message_grad_supported(a.chan), "mg_bee_message_grad_run: chan = %d is no multiple of 64", a.chan);
-    MG_REQUIRE(a.E >= 0 && a.E < (1L << 31) && a.n_src >= 0 && a.n_rows >= 0, "mg_bee_message_grad_run: bad size");
-    const bool left = a.d_0 || a.d_1 || a.d_2, right = a.d_enc != nullptr, vec = a.d_rh != nullptr;
-    MG_REQUIRE(!left || (a.d_0 && a.d_1 && a.d_2 && a.dst_row_ptr), "mg_bee_message_grad_run: the three operands' gradients come together");
-    hipStream_t st = (hipStream_t)stream;
-    const long slices = a.chan / 64, items = (long)a.n_src * slices, sums = (long)a.n_rows * slices;
-    MG_REQUIRE(items < (1L << 31) - 64 && sums < (1L << 31) - 64, "mg_bee_message_grad_run: too many nodes");
-    float *dl = static_cast<float*>(a.workspace), *part = dl + (left ? left_floats(a.E, a.chan) : 0);
-    if (a.E > 0 && (left || right || vec)) {
-        MG_REQUIRE(a.row_ptr && a.dst && a.rh && a.enc && a.l_0 && a.l_1 && a.l_2 && a.d_P0 && a.d_S1 && a.d_S2 && a.n_rows > 0 && (a.workspace || !(left || vec)),
-                   "mg_bee_message_grad_run: null pointer");
-        const long per_xcd = ceil_div(ceil_div(items, 4), kXcds);
-        if (left && right) launch<true, true>(a, vec, items, per_xcd, dl, part, st);
-        else if (left) launch<true, false>(a, vec, items, per_xcd, dl, part, st);
-        else if (right) launch<false, true>(a, vec, items, per_xcd, dl, part, st);
-        else launch<false, false>(a, vec, items, per_xcd, dl, part, st);
-        if (vec)
-            hipLaunchKernelGGL(bee_message_grad_rh_kernel, dim3((unsigned)ceil_div(3 * a.E, 256)), dim3(256), 0, st, part, 3 * a.E,
-                               (int)slices, a.d_rh);
+    return run<false>("mg_bee_message_grad_run", *args, stream);
+}
+
+int mg_bee_message_grad_rows_run(const mg_bee_message_grad_rows* args, mg_stream_t stream) {
+    MG_REQUIRE(args, "mg_bee_message_grad_rows_run: null pointer");
+    const mg_bee_message_grad_rows& r = *args;
+    mg_bee_message_grad a{};
+    a.l_0 = r.l_0; a.l_1 = r.l_1; a.l_2 = r.l_2; a.enc = r.enc; a.rh = r.rh;
+    // the products of a rank lie side by side, in the order 011 101 121 211 111 and 022 202 112 222 212
+    static const int s1[5] = {3, 4, 5, 6, 11}, s2[5] = {7, 8, 9, 10, 12};
+    for (int k = 0; k < 3; k++) a.dy[k] = r.d_P0 ? r.d_P0 + (long)k * r.chan : nullptr;
+    for (int k = 0; k < 5; k++) {
+        a.dy[s1[k]] = r.d_S1 ? r.d_S1 + (long)k * r.chan : nullptr;
+        a.dy[s2[k]] = r.d_S2 ? r.d_S2 + (long)k * r.chan : nullptr;
     }
-    if (left && sums > 0) {
-        const long per_xcd = ceil_div(ceil_div(sums, 4), kXcds);
-        hipLaunchKernelGGL(bee_message_grad_sum_kernel, dim3((unsigned)(per_xcd * kXcds)), dim3(256), 0, st, dl, a.dst_row_ptr, a.perm,
-                           sums, per_xcd, a.chan, a.d_0, a.d_1, a.d_2);
-    }
-    return check_launch("mg_bee_message_grad_run");
+    a.row_ptr = r.row_ptr; a.dst = r.dst; a.dst_row_ptr = r.dst_row_ptr; a.perm = r.perm;
+    a.E = r.E; a.n_src = r.n_src; a.n_rows = r.n_rows; a.chan = r.chan;
+    a.workspace = r.workspace;
+    a.d_0 = r.d_0; a.d_1 = r.d_1; a.d_2 = r.d_2; a.d_enc = r.d_enc; a.d_rh = r.d_rh;
+    return run<true>("mg_bee_message_grad_rows_run", a, stream);
 }
 
 }  // extern "C"

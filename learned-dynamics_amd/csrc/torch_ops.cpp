@@ -1374,12 +1374,41 @@ std::tuple<OptTensor, OptTensor, OptTensor> painn_grid_message_bwd(const at::Ten
     return {d_table, d_actv, d_v};
 }
 
-// gradients of the rank-0/1/2 message products: (l_0, l_1, l_2), enc, rh; see mg_bee_message_grad
+// gradients of the rank-0/1/2 message products: (l_0, l_1, l_2), enc, rh.  dy: three gradients, operands and products
+// component-major (mg_bee_message_grad_rows), or 13, all of them by channel (mg_bee_message_grad)
+template <typename Args>
+void bee_message_grad_fill(Args& a, const Tensors& left, Tensors& d_left, const at::Tensor& enc, const at::Tensor& rh,
+                           const at::Tensor& row_ptr, const at::Tensor& dst, const at::Tensor& dst_row_ptr, const OptTensor& perm,
+                           at::Tensor& ws, at::Tensor& d_enc, at::Tensor& d_rh) {
+    a.l_0 = fp(left[0]);
+    a.l_1 = fp(left[1]);
+    a.l_2 = fp(left[2]);
+    a.enc = fp(enc);
+    a.rh = fp(rh);
+    a.row_ptr = row_ptr.data_ptr<int>();
+    a.dst = dst.data_ptr<int>();
+    a.dst_row_ptr = dst_row_ptr.data_ptr<int>();
+    a.perm = perm.has_value() ? perm->data_ptr<int>() : nullptr;
+    a.E = enc.size(0);
+    a.n_src = (int)row_ptr.numel() - 1;
+    a.n_rows = (int)left[0].size(0);
+    a.chan = (int)enc.size(1);
+    a.workspace = ws.data_ptr();
+    if (!d_left.empty()) {
+        a.d_0 = fp(d_left[0]);
+        a.d_1 = fp(d_left[1]);
+        a.d_2 = fp(d_left[2]);
+    }
+    a.d_enc = d_enc.defined() ? fp(d_enc) : nullptr;
+    a.d_rh = d_rh.defined() ? fp(d_rh) : nullptr;
+}
+
 std::tuple<Tensors, OptTensor, OptTensor> bee_message_bwd(const Tensors& left, const at::Tensor& enc, const at::Tensor& rh,
                                                           const Tensors& dy, const at::Tensor& row_ptr, const at::Tensor& dst,
                                                           const at::Tensor& dst_row_ptr, const OptTensor& perm, bool want_left,
                                                           bool want_enc, bool want_rh) {
-    TORCH_CHECK(left.size() == 3 && dy.size() == 3, "bee_message_bwd: three operands and three gradients expected");
+    static const int rank_of[13] = {0, 0, 0, 1, 1, 1, 1, 2, 2, 2, 2, 1, 2};
+    TORCH_CHECK(left.size() == 3 && (dy.size() == 3 || dy.size() == 13), "bee_message_bwd: three operands and 3 or 13 gradients expected");
     check_input(enc, "enc");
     check_input(rh, "rh");
     check_input(row_ptr, "row_ptr", at::kInt);
@@ -1387,21 +1416,21 @@ std::tuple<Tensors, OptTensor, OptTensor> bee_message_bwd(const Tensors& left, c
     check_input(dst_row_ptr, "dst_row_ptr", at::kInt);
     if (perm.has_value()) check_input(*perm, "perm", at::kInt);
     TORCH_CHECK(enc.dim() == 2 && rh.dim() == 2, "bee_message_bwd: enc (edges, chan) and rh (edges, 3) expected");
+    const bool rows_layout = dy.size() == 3;
     const int64_t E = enc.size(0), C = enc.size(1), rows = left[0].size(0), n_src = row_ptr.numel() - 1;
-    const int64_t per_rank[3] = {C, 3 * C, 9 * C}, wanted[3] = {E * 3 * C, n_src * 15 * C, n_src * 45 * C};
+    const int64_t per_rank[3] = {C, 3 * C, 9 * C}, stacked[3] = {E * 3 * C, n_src * 15 * C, n_src * 45 * C};
     TORCH_CHECK(rh.numel() == 3 * E && dst.numel() == E && dst_row_ptr.numel() == rows + 1 && n_src >= 0 &&
                     (!perm.has_value() || perm->numel() == E),
                 "bee_message_bwd: operand sizes");
-    mg_bee_message_grad a{};
     for (int k = 0; k < 3; k++) {
         check_input(left[k], "left operand");
         TORCH_CHECK(left[k].numel() == rows * per_rank[k], "bee_message_bwd: operand sizes");
-        check_input(dy[k], "gradient of the products");
-        TORCH_CHECK(dy[k].numel() == wanted[k], "bee_message_bwd: gradient sizes");
     }
-    a.d_P0 = fp(dy[0]);
-    a.d_S1 = fp(dy[1]);
-    a.d_S2 = fp(dy[2]);
+    for (size_t k = 0; k < dy.size(); k++) {
+        check_input(dy[k], "gradient of the products");
+        TORCH_CHECK(dy[k].numel() == (rows_layout ? stacked[k] : (rank_of[k] ? n_src : E) * per_rank[rank_of[k]]),
+                    "bee_message_bwd: gradient sizes");
+    }
     c10::hip::HIPGuardMasqueradingAsCUDA guard(enc.device());
     Tensors d_left;
     if (want_left)
@@ -1412,28 +1441,19 @@ std::tuple<Tensors, OptTensor, OptTensor> bee_message_bwd(const Tensors& left, c
     size_t bytes = 0;
     check(mg_bee_message_grad_workspace_bytes(E, (int)C, want_left, want_rh, &bytes));
     at::Tensor ws = bytes_like(enc, bytes);
-    a.l_0 = fp(left[0]);
-    a.l_1 = fp(left[1]);
-    a.l_2 = fp(left[2]);
-    a.enc = fp(enc);
-    a.rh = fp(rh);
-    a.row_ptr = row_ptr.data_ptr<int>();
-    a.dst = dst.data_ptr<int>();
-    a.dst_row_ptr = dst_row_ptr.data_ptr<int>();
-    a.perm = perm.has_value() ? perm->data_ptr<int>() : nullptr;
-    a.E = E;
-    a.n_src = (int)n_src;
-    a.n_rows = (int)rows;
-    a.chan = (int)C;
-    a.workspace = ws.data_ptr();
-    if (want_left) {
-        a.d_0 = fp(d_left[0]);
-        a.d_1 = fp(d_left[1]);
-        a.d_2 = fp(d_left[2]);
+    if (rows_layout) {
+        mg_bee_message_grad_rows a{};
+        bee_message_grad_fill(a, left, d_left, enc, rh, row_ptr, dst, dst_row_ptr, perm, ws, d_enc, d_rh);
+        a.d_P0 = fp(dy[0]);
+        a.d_S1 = fp(dy[1]);
+        a.d_S2 = fp(dy[2]);
+        check(mg_bee_message_grad_rows_run(&a, stream_of(enc)));
+    } else {
+        mg_bee_message_grad a{};
+        bee_message_grad_fill(a, left, d_left, enc, rh, row_ptr, dst, dst_row_ptr, perm, ws, d_enc, d_rh);
+        for (int k = 0; k < 13; k++) a.dy[k] = fp(dy[k]);
+        check(mg_bee_message_grad_run(&a, stream_of(enc)));
     }
-    a.d_enc = want_enc ? fp(d_enc) : nullptr;
-    a.d_rh = want_rh ? fp(d_rh) : nullptr;
-    check(mg_bee_message_grad_run(&a, stream_of(enc)));
     return {d_left, want_enc ? OptTensor(d_enc) : OptTensor(), want_rh ? OptTensor(d_rh) : OptTensor()};
 }
 

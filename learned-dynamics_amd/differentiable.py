@@ -994,11 +994,11 @@ class _MessageProducts(torch.autograd.Function):
         if enc_source is not None:
             enc8, W, b = enc_source
             b = b if b is not None else torch.zeros(C, dtype=torch.float32, device=enc.device)
-            *stacked, node_max, edge_max = ops.bee_message(by_src.row_ptr, by_dst.index, rh, enc8.contiguous(),
-                                                           *(_by_component(*left) if by_label else left),
-                                                           W.detach().contiguous(), b.detach().contiguous(), want_node_max=True)
+            operands = by_src.row_ptr, by_dst.index, rh, enc8.contiguous(), *(_by_component(*left) if by_label else left)
+            weights = W.detach().contiguous(), b.detach().contiguous()
             if by_label:
-                return ops.unstack_products(*stacked)
+                return ops.unstack_products(*ops.bee_message(*operands, *weights))
+            *stacked, node_max, edge_max = ops.bee_message(*operands, *weights, want_node_max=True)
         else:
             phi_v, phi_d = ops.bee_edge_filters_fwd(enc, rh)
             prods = ops.bee_fwd_indexed(*(left if by_label else (t.contiguous() for t in _by_channel(*left))), by_dst.index, enc,

@@ -581,6 +581,8 @@ def bee_message_grad(left, enc, rh, d_products, by_src, by_dst, want_left, want_
     """Gradients of bee_message for the node operands `left` (nodes, chan), (nodes, 3, chan), (nodes, 9, chan), read at the edges'
     destinations, and for enc (edges, chan) and rh (edges, 3), which the edge filters are made of: ([d_l0, d_l1, d_l2] or
     [], d_enc or None, d_rh or None).  d_products: those of P0, S1 and S2."""
+    if len(d_products) != 3:
+        raise RuntimeError("the gradients of P0, S1 and S2 expected")
     return _ext.bee_message_bwd(list(left), enc, rh, list(d_products), by_src.row_ptr, by_dst.index, by_dst.row_ptr, by_dst.perm,
                                 bool(want_left), bool(want_enc), bool(want_rh))
 
@@ -588,10 +590,10 @@ def bee_message_grad(left, enc, rh, d_products, by_src, by_dst, want_left, want_
 def bee_message_bwd(left, enc, rh, dys, by_src, by_dst, want_left, want_enc, want_rh):
     """bee_message_grad with the operands and their gradients as (nodes, chan, 3, ..) and those of the 13 products one by one, in
     BEE_ORDER: one row per edge for the scalar products, one per source node for the others (their sums over its edges)."""
-    n, chan = left[0].shape
-    by_comp = [left[0]] + [t.reshape(n, chan, -1).transpose(1, 2).contiguous() for t in left[1:]]
-    d_left, d_enc, d_rh = bee_message_grad(by_comp, enc, rh, stack_products(dys), by_src, by_dst, want_left, want_enc, want_rh)
-    return [d.transpose(1, 2).reshape(t.shape) if d.dim() == 3 else d for d, t in zip(d_left, left)], d_enc, d_rh
+    if len(dys) != 13:
+        raise RuntimeError("the gradients of 13 products expected")
+    return _ext.bee_message_bwd(list(left), enc, rh, list(dys), by_src.row_ptr, by_dst.index, by_dst.row_ptr, by_dst.perm,
+                                bool(want_left), bool(want_enc), bool(want_rh))
 
 
 def stack_products(prods):

@@ -83,3 +83,27 @@ def test_torch_binding_loads_and_exports_the_reference_names():
         assert "must be a CUDA tensor" in str(e)
     else:
         raise AssertionError("a host tensor was accepted")
+
+
+def test_message_gradient_takes_the_struct_with_a_pointer_per_product():
+    """mg_bee_message_grad (include/managan_hip.h): 13 gradients by product and then the graph, as callers in C lay it out.  With one
+    gradient missing the call names it and launches nothing (the other pointers are never followed)."""
+    import ctypes
+    L = importlib.import_module("learned-dynamics_amd._lib")
+    lib = L.load()
+
+    class Args(ctypes.Structure):
+        _fields_ = [(n, ctypes.c_void_p) for n in ("l_0", "l_1", "l_2", "enc", "rh")] + [("dy", ctypes.c_void_p * 13)] + \
+                   [(n, ctypes.c_void_p) for n in ("row_ptr", "dst", "dst_row_ptr", "perm")] + [("E", ctypes.c_long)] + \
+                   [(n, ctypes.c_int) for n in ("n_src", "n_rows", "chan")] + \
+                   [(n, ctypes.c_void_p) for n in ("workspace", "d_0", "d_1", "d_2", "d_enc", "d_rh")]
+
+    for missing in (0, 7, 12):
+        a = Args(E=10, n_src=3, n_rows=4, chan=64)
+        for name, kind in Args._fields_:
+            if kind is ctypes.c_void_p:
+                setattr(a, name, 16)
+        for k in range(13):
+            a.dy[k] = None if k == missing else 16
+        assert lib.mg_bee_message_grad_run(ctypes.byref(a), None) != 0
+        assert f"gradient {missing} is null" in lib.mg_last_error().decode()

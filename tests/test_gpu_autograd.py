@@ -1261,3 +1261,22 @@ def test_rank012_layers_on_stacked_products(pkg, chan, dims, N, E):
             if x is not None:
                 assert x.shape == y.shape
                 assert float((x - y).abs().max()) <= 1e-5 * max(float(y.abs().max()), 1e-3), (type(module).__name__, k)
+
+
+@pytest.mark.parametrize("N,E,C", [(5, 3, 64), (37, 500, 192)])
+def test_message_gradients_by_product_and_by_component(pkg, ops, N, E, C):
+    """ops.bee_message_bwd, operands and products one by one and by channel, and ops.bee_message_grad, component-major and side
+    by side: one kernel in two layouts, the same sums in the same order."""
+    gl = importlib.import_module("learned-dynamics_amd.graph_layers")
+    g = torch.Generator().manual_seed(E)
+    rnd = lambda *shape: torch.randn(*shape, generator=g).cuda()
+    src = torch.sort(torch.randint(0, N, (E,), generator=g)).values
+    graph = gl.Graph(src.cuda(), torch.randint(0, N, (E,), generator=g).cuda(), None, 1, N)
+    left, enc, rh = [rnd(N, C, *([3] * k)) for k in range(3)], rnd(E, C), rnd(E, 3)
+    dys = [rnd(E if lab[2] == "0" else N, C, *([3] * int(lab[2]))) for lab in ops.BEE_ORDER]
+    by_comp = [left[0]] + [t.flatten(2).transpose(1, 2).contiguous() for t in left[1:]]
+    d_left, *rest = ops.bee_message_bwd(left, enc, rh, dys, graph.by_src, graph.by_dst, True, True, True)
+    d_rows, *rest_rows = ops.bee_message_grad(by_comp, enc, rh, ops.stack_products(dys), graph.by_src, graph.by_dst, True, True, True)
+    for a, b in zip(d_left, d_rows):
+        assert torch.equal(a.flatten(2).transpose(1, 2) if a.dim() > 2 else a, b)
+    assert all(torch.equal(a, b) for a, b in zip(rest, rest_rows))
