@@ -1037,8 +1037,8 @@ class _MessageProducts(torch.autograd.Function):
                 leaves = [t if t.requires_grad else t.detach().requires_grad_() for t in saved]
                 out = _message_products_plain(*(leaves[:3] if by_label else _by_channel(*leaves[:3])), *leaves[3:], by_dst, by_src)
                 out = out if by_label else _as_rows(*ops.stack_products(out))
-                out, dys = zip(*((o, g) for o, g in zip(out, dys) if g is not None))
-                grads = torch.autograd.grad(out, leaves, dys, create_graph=True, allow_unused=True)
+                dys = [torch.zeros_like(o) if g is None else g for o, g in zip(out, dys)]
+                grads = torch.autograd.grad(out, leaves, dys, create_graph=True)
             return tuple(g if nd else None for g, nd in zip(grads, need)) + (None, None, None, None)
         *left, enc, rh = saved
         N, C, E = left[0].shape[0], left[0].shape[1], enc.shape[0]
@@ -1082,8 +1082,8 @@ class _NodeProducts(torch.autograd.Function):
             with torch.enable_grad():
                 leaves = [t if t.requires_grad else t.detach().requires_grad_() for t in operands]
                 out = _as_rows(*ops.stack_products(Bee.apply(*_by_channel(*leaves))))
-                out, dys = zip(*((o, g) for o, g in zip(out, dys) if g is not None))
-                grads = torch.autograd.grad(out, leaves, dys, create_graph=True, allow_unused=True)
+                dys = [torch.zeros_like(o) if g is None else g for o, g in zip(out, dys)]
+                grads = torch.autograd.grad(out, leaves, dys, create_graph=True)
         else:
             N, C = operands[0].shape
             shapes = (N, 3, C), (N, 3, 5, C), (N, 9, 5, C)

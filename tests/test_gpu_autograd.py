@@ -1280,3 +1280,37 @@ def test_message_gradients_by_product_and_by_component(pkg, ops, N, E, C):
     for a, b in zip(d_left, d_rows):
         assert torch.equal(a.flatten(2).transpose(1, 2) if a.dim() > 2 else a, b)
     assert all(torch.equal(a, b) for a, b in zip(rest, rest_rows))
+
+
+@pytest.mark.parametrize("what", ["by product", "rows", "node products"])
+def test_recorded_backward_without_any_gradient(pkg, what):
+    """The functions of the rank-0/1/2 products behind one whose backward returns no gradient: autograd calls them with None for
+    every result, and a recorded backward pass gives zeros, as the plain one does."""
+    diff, gl = (importlib.import_module(f"learned-dynamics_amd.{m}") for m in ("differentiable", "graph_layers"))
+    g = torch.Generator().manual_seed(3)
+    N, E, C = 9, 20, 256
+    src = torch.sort(torch.randint(0, N, (E,), generator=g)).values
+    graph = gl.Graph(src.cuda(), torch.randint(0, N, (E,), generator=g).cuda(), None, 1, N)
+    rnd = lambda *shape: torch.randn(*shape, generator=g).cuda().requires_grad_()
+    rows = lambda: [rnd(N, C), rnd(N, 3, C), rnd(N, 9, C)]
+    if what == "node products":
+        leaves = rows() + rows()
+        out = diff._NodeProducts.apply(*leaves)[:3]
+    else:
+        leaves = (rows() if what == "rows" else [rnd(N, C, *[3] * k) for k in range(3)]) + [rnd(E, C), rnd(E, 3)]
+        out = diff._MessageProducts.apply(*leaves, graph.by_dst, graph.by_src, None, what == "by product")
+        out = out[:3] if what == "rows" else out
+
+    class Drop(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, *ts):
+            return sum(t.sum() for t in ts)
+
+        @staticmethod
+        def backward(ctx, g):
+            return (None,) * len(out)
+
+    dropped = Drop.apply(*out)
+    for recorded in (False, True):
+        grads = torch.autograd.grad(dropped, leaves, retain_graph=True, create_graph=recorded)
+        assert all(float(t.abs().max()) == 0.0 for t in grads)
