@@ -1982,8 +1982,9 @@ def tensor_linear_f16x2_rowsum(W, x, x_bound, row_ptr, seg, n_out, bias=None, ac
 
 def mlp_rowsum_supported(rows, dim_in, dim, x):
     """mlp_leaky_rowsum takes these sizes.  Below 4096 rows (64 workgroups) a linear that splits its reduction and a plain
-    segment sum stay; from there on the one kernel is faster at every size (4096 rows: 256 -> 512 38 against 52 us, 32 -> 64 17 and 20)."""
-    return (get_linear_mode() == LINEAR_F16X2 and rows >= 4096 and x.data_ptr() % 16 == 0
+    segment sum stay; from there on the one kernel is faster at every size (4096 rows: 256 -> 512 38 against 52 us).  A linear of
+    fewer than 64 columns has fp32 arithmetic, here as everywhere."""
+    return (get_linear_mode() == LINEAR_F16X2 and rows >= 4096 and dim_in >= 64 and dim >= 64 and x.data_ptr() % 16 == 0
             and bool(_lib.mg_mlp_f16x2_supported(int(dim_in), int(dim))))
 
 

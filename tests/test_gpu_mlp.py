@@ -1,4 +1,6 @@
 """Linear, SiLU, Linear, SiLU, Linear as one kernel (csrc/mlp_f16x2.hip) against the same formula in float64."""
+import importlib
+
 import pytest
 import torch
 
@@ -6,6 +8,11 @@ pytestmark = pytest.mark.gpu
 
 ACTS = (1, 1, 0)
 INF, NAN = float("inf"), float("nan")
+
+
+@pytest.fixture
+def bee(pkg):
+    return importlib.import_module("learned-dynamics_amd.bee_layers")
 
 
 def _weights(dim_in, dim, seed=3):
@@ -176,6 +183,44 @@ def test_mlp_summed_over_segments(ops, rows, dim_in, dim):
         big, size = _layers_and_sum(x.double(), W, b, seg, n_out)
         k = seg[rows // 2]
         assert float((odd[k].double() - big[k]).norm() / size[k]) <= 1.5e-6
+
+
+def _summed(pkg, dim, rows, bias_offset=0):
+    """bee_layers.MLP of `dim` columns, rows and their segments, and the sum of the MLP's rows in float32 and float64."""
+    torch.manual_seed(dim)
+    mlp = pkg.MLP(dim).cuda()
+    for k in (0, 2):
+        layer = mlp.layers[k]
+        flat = torch.zeros(bias_offset + layer.out_features, device="cuda")
+        flat[bias_offset:] = layer.bias.detach()
+        layer.bias = torch.nn.Parameter(flat[bias_offset:])
+    x = torch.randn(rows, dim, generator=torch.Generator().manual_seed(rows)).cuda()
+    row_ptr, seg = (t.int().cuda() for t in _segments(rows, dim))
+    n_out = row_ptr.numel() - 1
+
+    def reference(dt):
+        w = lambda t: t.detach().to(dt)
+        W, b = [w(mlp.layers[k].weight) for k in (0, 2, 4)], [w(mlp.layers[k].bias) for k in (0, 2, 4)]
+        s_h, _ = _layers_and_sum(x.to(dt), W, b, seg.long(), n_out)
+        s_x = torch.zeros(n_out, dim, dtype=dt, device="cuda").index_add(0, seg.long(), x.to(dt))
+        count = (row_ptr[1:] - row_ptr[:-1]).to(dt)[:, None]
+        return s_x @ w(mlp.lin_direct.weight).t() + s_h @ W[2].t() + count * b[2]
+
+    with torch.no_grad():
+        got = mlp.summed_over_rows(x, row_ptr, n_out, seg=seg)
+    ref = reference(torch.float64)
+    error = lambda y: float((y.double() - ref).norm() / ref.norm())
+    return error(got), error(reference(torch.float32))
+
+
+def test_narrow_layers_summed_over_segments_stay_in_fp32(bee, ops, monkeypatch):
+    """A linear of 32 columns has fp32 arithmetic: the kernel of 22-bit pieces takes a layer from 64 columns on."""
+    x = torch.zeros(5000, 64).cuda()
+    assert ops.mlp_rowsum_supported(5000, 64, 64, x)
+    assert not ops.mlp_rowsum_supported(5000, 32, 64, x) and not ops.mlp_rowsum_supported(5000, 64, 32, x)
+    monkeypatch.setattr(ops, "mlp_leaky_rowsum", None)
+    err, f32 = _summed(bee, 32, 5000)
+    assert err <= 2 * f32                                        # (two fp32 sums of the same terms in different orders)
 
 
 @pytest.mark.parametrize("rows, dim_in, dim, dim_out", [(256, 64, 64, 32), (257, 96, 96, 160), (700, 256, 512, 256),
