@@ -259,7 +259,7 @@ class MLP(nn.Module):
         W_last = W_last0 if scale == 1.0 else _derived(self, ("last_scaled", scale), (W_last0,), lambda: scale * W_last0)
         b_last = b_last0 if scale == 1.0 else _derived(self, ("last_bias_scaled", scale), (b_last0,), lambda: scale * b_last0)
         L = self.layers
-        if seg is not None and ops.mlp_rowsum_supported(x.shape[0], L[0].in_features, L[0].out_features, x):
+        if seg is not None and ops.mlp_rowsum_supported(x.shape[0], L[0].in_features, L[0].out_features, x, L[0].bias, L[2].bias):
             s_h = ops.mlp_leaky_rowsum(L[0].weight, L[0].bias, L[2].weight, L[2].bias, x, row_ptr, seg, n_out)
         else:
             if bound is None and ops.get_linear_mode() == ops.LINEAR_F16X2:

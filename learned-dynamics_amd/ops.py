@@ -1980,11 +1980,12 @@ def tensor_linear_f16x2_rowsum(W, x, x_bound, row_ptr, seg, n_out, bias=None, ac
     return out, y
 
 
-def mlp_rowsum_supported(rows, dim_in, dim, x):
+def mlp_rowsum_supported(rows, dim_in, dim, x, *biases):
     """mlp_leaky_rowsum takes these sizes.  Below 4096 rows (64 workgroups) a linear that splits its reduction and a plain
     segment sum stay; from there on the one kernel is faster at every size (4096 rows: 256 -> 512 38 against 52 us).  A linear of
-    fewer than 64 columns has fp32 arithmetic, here as everywhere."""
-    return (get_linear_mode() == LINEAR_F16X2 and rows >= 4096 and dim_in >= 64 and dim >= 64 and x.data_ptr() % 16 == 0
+    fewer than 64 columns has fp32 arithmetic, here as everywhere.  The kernel reads x and the biases 16 bytes at a time."""
+    return (get_linear_mode() == LINEAR_F16X2 and rows >= 4096 and dim_in >= 64 and dim >= 64
+            and all(t is None or t.data_ptr() % 16 == 0 for t in (x, *biases))
             and bool(_lib.mg_mlp_f16x2_supported(int(dim_in), int(dim))))
 
 

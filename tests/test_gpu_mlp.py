@@ -223,6 +223,18 @@ def test_narrow_layers_summed_over_segments_stay_in_fp32(bee, ops, monkeypatch):
     assert err <= 2 * f32                                        # (two fp32 sums of the same terms in different orders)
 
 
+def test_biases_at_any_offset_summed_over_segments(bee, ops, monkeypatch):
+    """Biases that are views of a flat buffer: layer by layer, as before there was a kernel for both; that kernel takes the others."""
+    rows = 4200
+    called, kernel = [], ops.mlp_leaky_rowsum
+    monkeypatch.setattr(ops, "mlp_leaky_rowsum", lambda *a: (called.append(1), kernel(*a))[1])
+    for offset in (0, 1, 4):
+        err, f32 = _summed(bee, 96, rows, bias_offset=offset)
+        assert err <= 1.5e-6
+        assert len(called) == (0 if offset % 4 else 1), offset
+        called.clear()
+
+
 @pytest.mark.parametrize("rows, dim_in, dim, dim_out", [(256, 64, 64, 32), (257, 96, 96, 160), (700, 256, 512, 256),
                                                          (5000, 64, 128, 64)])
 def test_leaky_mlp_and_its_adjoint(ops, rows, dim_in, dim, dim_out):
