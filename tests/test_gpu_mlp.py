@@ -121,6 +121,25 @@ def test_mlp_adjoint_in_one_kernel(ops, rows, dim_in, dim, dual):
     assert no_x is None
 
 
+@pytest.mark.parametrize("spread", [0.3, 1.0, 4.0])
+def test_silu_between_the_layers(ops, spread):
+    """The hidden rows h = SiLU(z) that the training kernel keeps beside z, entry by entry in float64, against the same from float32
+    exp and a division: no further off.  And the ends of the range: four roundings of 2^-24 and an exponential good to one more."""
+    W, b = _weights(64, 256)
+    x = spread * 1.4 * torch.randn(4000, 64, generator=torch.Generator().manual_seed(3)).cuda()
+    _, _, saved = ops.mlp_silu_fwd(x, None, None, W, b, True)
+    z, h = saved[1], saved[3]
+    ref = torch.nn.functional.silu(z.double())
+    rms = lambda y: float((((y.double() - ref) / ref) ** 2).mean().sqrt())
+    assert rms(h) <= rms(z * (1.0 / (1.0 + torch.exp(-z)))), spread
+    bias = torch.tensor([200.0, 87.0, 0.0, -87.0, -89.0, -200.0, -1e30, 1e30]).repeat(8).cuda()
+    _, _, saved = ops.mlp_silu_fwd(torch.zeros(64, 64).cuda(), None, None, [W[0][:64]] + [w[:64, :64].contiguous() for w in W[1:]],
+                                   [bias] + [t[:64].contiguous() for t in b[1:]], True)
+    ref = torch.nn.functional.silu(bias.double())
+    # (where the sigmoid is below the smallest normal number, 2^-126, the result is 0: off by 89 * 2^-126 = 1e-36 at most)
+    assert bool(((saved[3].double() - ref).abs() <= 3e-7 * ref.abs() + 1.1e-36).all())
+
+
 @pytest.mark.parametrize("rows, dim", [(50, 64), (1100, 512), (8300, 512)])
 def test_mlp_adjoint_of_a_row_beyond_the_pieces(ops, rows, dim):
     W, b = _weights(64, dim)
