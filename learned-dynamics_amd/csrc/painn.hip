@@ -285,6 +285,15 @@ __global__ void __launch_bounds__(256) painn_no_edges_kernel(long count, const f
     for (long t = (long)blockIdx.x * 256 + threadIdx.x; t < count; t += (long)gridDim.x * 256) out[t] = res ? res[t] : 0.f;
 }
 
+__device__ __forceinline__ void grid_slice_to_lds(float* tab, const float* __restrict__ table, int tab_rows, int n, int slice) {
+    for (int q = threadIdx.x; q < (tab_rows + kSliceExtraRows) * (kSliceCols / 4); q += blockDim.x) {
+        const int row = q / (kSliceCols / 4), piece = q % (kSliceCols / 4), k = piece / 4, c4 = piece % 4;
+        st4(tab + row * kSliceRowF + 4 * piece,
+            ld4(table + (long)(row & (tab_rows - 1)) * 4 * n + k * n + slice * kSliceChan + 4 * c4));
+    }
+    __syncthreads();
+}
+
 // Twelve waves on a CU: the rows of the next 16 edges and the indices of those after them are on their way while a step is computed,
 // which takes 140 registers.  16 384 nodes, 1.6 M edges, n = 128: 410 -> 360 us; before, sixteen waves without it (a node's first rows,
 // records and indices were three waits in a row).  In 128 registers 30 of them spill; eight waves 409 us; all four
@@ -302,12 +311,7 @@ __global__ void __launch_bounds__(kTableThreads) painn_table_message_lds_kernel(
     // ever holds that slice's columns of the node rows
     const int slice = blockIdx.x % n_slices;
     const int group = blockIdx.x / n_slices, groups = gridDim.x / n_slices;
-    for (int q = threadIdx.x; q < (tab_rows + kSliceExtraRows) * (kSliceCols / 4); q += blockDim.x) {
-        const int row = q / (kSliceCols / 4), piece = q % (kSliceCols / 4), k = piece / 4, c4 = piece % 4;
-        st4(tab + row * kSliceRowF + 4 * piece,
-            ld4(table + (long)(row & (tab_rows - 1)) * 4 * n + k * n + slice * kSliceChan + 4 * c4));
-    }
-    __syncthreads();
+    grid_slice_to_lds(tab, table, tab_rows, n, slice);
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), waves = blockDim.x / kWave;
     const int l4 = lane & 3, sub = lane >> 2;                 // 4 channels of edge `sub` of the step
     // 32-bit element offsets (the host checks that they fit) keep the address arithmetic short
@@ -411,6 +415,82 @@ __global__ void __launch_bounds__(kTableThreads) painn_table_message_lds_kernel(
         if (s0.node < 0) return;
         step(odd, even);
         if (s0.node < 0) return;
+    }
+}
+
+// The same with sixteen waves on a CU and nothing requested ahead but an edge's record, for few nodes (the same sums in the same
+// order): their rows come out of the L2 soon enough, and what counts is how many nodes the waves take in turn.
+constexpr int kFewThreads = 1024, kFewTurns = 5;
+__global__ void __launch_bounds__(kFewThreads) painn_table_message_lds_few_kernel(
+    const int* __restrict__ row_ptr, const int* __restrict__ dst, const int* __restrict__ node_order, long n_nodes,
+    const float4* __restrict__ rec, const float* __restrict__ table, int tab_rows, const float* __restrict__ actv_s,
+    const float* __restrict__ x_v, int n, const float* __restrict__ res_a, const float* __restrict__ res_v,
+    float* __restrict__ out_a, float* __restrict__ out_v, long n_edges) {
+    extern __shared__ float tab[];                            // (tab_rows + 3) x kSliceRowF
+    const int n_slices = n / kSliceChan, slice = blockIdx.x % n_slices;
+    const int group = blockIdx.x / n_slices, groups = gridDim.x / n_slices;
+    grid_slice_to_lds(tab, table, tab_rows, n, slice);
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, waves = blockDim.x / kWave;
+    const int l4 = lane & 3, sub = lane >> 2;                 // 4 channels of edge `sub` of the step
+    const unsigned a_stride = (unsigned)n_slices * kSliceCols, v_stride = 3u * (unsigned)n, last_node = (unsigned)(n_nodes - 1);
+    const float* a_base = actv_s + slice * kSliceCols + 4 * l4;
+    const float* v_base = x_v + (slice * kSliceChan + 4 * l4) * 3;
+    const float* tab_l = tab + 4 * l4;
+    const bool is_a = sub >= 12;                              // (as above: lanes 12 .. 15 hold the scalar sums)
+    const long o_lane = slice * kSliceChan + 4 * l4;
+    for (long slot = (long)group * waves + wave; slot < n_nodes; slot += (long)groups * waves) {
+        const long node = node_order ? node_order[slot] : slot;
+        const int lo = max(row_ptr[node], 0), hi = (int)min((long)row_ptr[node + 1], n_edges);
+        float acc[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) acc[k] = 0.f;
+        int e = lo + sub;
+        unsigned j = 0;
+        float4 ra = make_float4(0.f, 0.f, 0.f, 0.f), rb = ra;
+        if (e < hi) { j = min((unsigned)dst[e], last_node); ra = rec[2 * (long)e]; rb = rec[2 * (long)e + 1]; }
+        while (e < hi) {
+            const float* a_row = a_base + j * a_stride;
+            const float* v_row = v_base + j * v_stride;
+            float4 a[4], v[3];
+#pragma unroll
+            for (int k = 0; k < 4; k++) a[k] = ld4(a_row + k * kSliceChan);
+#pragma unroll
+            for (int k = 0; k < 3; k++) v[k] = ld4(v_row + 4 * k);
+            e += 16;
+            unsigned j_next = 0;
+            float4 na = ra, nb = rb;
+            if (e < hi) { j_next = min((unsigned)dst[e], last_node); na = rec[2 * (long)e]; nb = rec[2 * (long)e + 1]; }
+            const float* tp = tab_l + __float_as_int(ra.x);
+            const float w0 = ra.y, w1 = ra.z, w2 = ra.w, w3 = rb.x, ux = rb.y, uy = rb.z, uz = rb.w;
+            float p[4][4];                                    // filter x activation: block k, channel c
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float4 t0 = ld4(tp + k * kSliceChan), t1 = ld4(tp + kSliceRowF + k * kSliceChan),
+                             t2 = ld4(tp + 2 * kSliceRowF + k * kSliceChan), t3 = ld4(tp + 3 * kSliceRowF + k * kSliceChan);
+                p[k][0] = (w0 * t0.x + w1 * t1.x + w2 * t2.x + w3 * t3.x) * a[k].x;
+                p[k][1] = (w0 * t0.y + w1 * t1.y + w2 * t2.y + w3 * t3.y) * a[k].y;
+                p[k][2] = (w0 * t0.z + w1 * t1.z + w2 * t2.z + w3 * t3.z) * a[k].z;
+                p[k][3] = (w0 * t0.w + w1 * t1.w + w2 * t2.w + w3 * t3.w) * a[k].w;
+            }
+            const float vv[12] = {v[0].x, v[0].y, v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w,
+                                  v[2].x, v[2].y, v[2].z, v[2].w};
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const float x = vv[3 * c], y = vv[3 * c + 1], z = vv[3 * c + 2];
+                const float cx = y * uz - z * uy, cy = z * ux - x * uz, cz = x * uy - y * ux;   // v x u
+                acc[3 * c + 0] = fmaf(ux, p[2][c], fmaf(cx, p[1][c], fmaf(x, p[0][c], acc[3 * c + 0])));
+                acc[3 * c + 1] = fmaf(uy, p[2][c], fmaf(cy, p[1][c], fmaf(y, p[0][c], acc[3 * c + 1])));
+                acc[3 * c + 2] = fmaf(uz, p[2][c], fmaf(cz, p[1][c], fmaf(z, p[0][c], acc[3 * c + 2])));
+                acc[12 + c] += p[3][c];
+            }
+            j = j_next; ra = na; rb = nb;
+        }
+        const long o = node * n + o_lane;
+        float sum = sum_over_slots(acc, lane);
+        float* outp = is_a ? out_a + o + (sub - 12) : out_v + o * 3 + sub;
+        const float* resp = is_a ? (res_a ? res_a + o + (sub - 12) : nullptr) : (res_v ? res_v + o * 3 + sub : nullptr);
+        if (resp) sum += *resp;
+        *outp = sum;
     }
 }
 
@@ -685,13 +765,19 @@ int mg_painn_table_message_sliced(const int* row_ptr, const int* dst, const int*
     const int n_slices = n / kSliceChan;
     const size_t lds_bytes = (size_t)(table_rows + kSliceExtraRows) * kSliceRowF * sizeof(float);
     // more than 64 KB of dynamic LDS has to be asked for (per device, so on every call)
-    MG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(painn_table_message_lds_kernel),
-                               hipFuncAttributeMaxDynamicSharedMemorySize,
+    const long groups = ceil_div(256, n_slices);              // one workgroup per CU
+    // Which kernel: a node in turn of a wave costs 3/4 as much with twelve waves a CU as with sixteen, and the first one half a node
+    // more.  From six in turn on the twelve are as fast or faster, and by 10 to 15 % where the L2 does not hold the nodes' rows.  us,
+    // sixteen / twelve waves, n = 128: 500 nodes of 51 edges 15.3 / 18.6, 640 21.1 / 20.0, 1024 23.5 / 26.1, 2048 of 99 edges
+    // 63 / 68, 3000 89.8 / 86.3, 16 384 of 89 410 / 367; n = 64: 4096 of 99 64.1 / 67.6, 8192 122 / 115.
+    const long turns = ceil_div(n_nodes, groups * (kFewThreads / kWave)), turns_12 = ceil_div(n_nodes, groups * (kTableThreads / kWave));
+    const bool few = turns <= kFewTurns && 15 * turns < 5 + 11 * turns_12;
+    const auto kernel = few ? painn_table_message_lds_few_kernel : painn_table_message_lds_kernel;
+    const int threads = few ? kFewThreads : kTableThreads;
+    MG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                (kSliceMaxRows + kSliceExtraRows) * kSliceRowF * (int)sizeof(float)));
-    long groups = ceil_div(256, n_slices);                    // one workgroup per CU
-    const long max_groups = ceil_div(n_nodes, 16);
-    if (groups > max_groups) groups = max_groups;
-    hipLaunchKernelGGL(painn_table_message_lds_kernel, dim3((unsigned)(groups * n_slices)), dim3(kTableThreads), lds_bytes,
+    const long max_groups = ceil_div(n_nodes, threads / kWave);      // (a node to a wave while there are CUs left)
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((groups < max_groups ? groups : max_groups) * n_slices)), dim3(threads), lds_bytes,
                        (hipStream_t)stream, row_ptr, dst, node_order, (long)n_nodes,
                        reinterpret_cast<const float4*>(records), table, table_rows, actv_sliced, x_v, n, res_a, res_v,
                        out_a, out_v, n_edges);

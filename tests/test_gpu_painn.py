@@ -682,6 +682,36 @@ def test_message_with_the_grid_in_lds_over_nodes_of_any_degree(pkg, degrees, ord
             assert float((x - y).abs().max()) <= 2 ** -24 * (8 * max(1, max(degrees)) ** 0.5 + rows) * max(1.0, float(y.abs().max()))
 
 
+@pytest.mark.parametrize("degrees", [(0,), (0, 0, 1), (16, 0, 15, 17, 0, 33, 32, 1), (0, 100, 0), tuple(range(0, 70))])
+@pytest.mark.parametrize("ordered", [False, True])
+def test_messages_of_few_and_of_many_nodes(pkg, degrees, ordered):
+    """A call with few nodes, a wave for each, and one with more than two rounds of them have a kernel each: the same sums in the same
+    order, bit for bit, and both as the kernel that reads the grid from memory (tolerance above)."""
+    ops = importlib.import_module("learned-dynamics_amd.ops")
+    gen = torch.Generator().manual_seed(len(degrees))
+    n, rows, few, many, period = 32, 64, 1000, 2100, 10.0        # (two slices: 128 workgroups each, sixteen or twelve waves)
+    deg = torch.tensor(degrees).repeat(-(-many // len(degrees)))[:many]
+    row_ptr = torch.cat([torch.zeros(1, dtype=torch.int64), deg.cumsum(0)]).int().cuda()
+    E = int(row_ptr[-1])
+    dst = torch.cat([torch.randint(0, few - 1, (E,), generator=gen), torch.full((5,), 2 ** 31 - 1)]).int().cuda()
+    r = torch.randn(E + 5, 3, generator=gen).cuda() * 2
+    table, actv, v = (torch.randn(*s, generator=gen).cuda() for s in ((rows, 4 * n), (many, 4 * n), (many, n, 3)))
+    actv[few - 1], v[few - 1] = float("inf"), float("nan")
+    res_a, res_v = torch.randn(many, n, generator=gen).cuda(), torch.randn(many, n, 3, generator=gen).cuda()
+    perm = ops.painn_slice_permutation(n, "cuda")
+
+    def message(N, res):
+        order = torch.randperm(N, generator=gen).int().cuda() if ordered else None
+        return ops.painn_table_message_sliced(row_ptr[:N + 1], dst, r, table, period, actv[:N, perm].contiguous(), v[:N].contiguous(), 0.1,
+                                              *(t if t is None else t[:N].contiguous() for t in res), node_order=order)
+
+    for res in ((None, None), (res_a, res_v)):
+        want = ops.painn_table_message(row_ptr, dst, r, table, period, actv, v, 0.1, *res)
+        for small, big, y in zip(message(few, res), message(many, res), want):
+            assert torch.equal(big[:few], small)
+            assert float((big - y).abs().max()) <= 2 ** -24 * (8 * max(1, max(degrees)) ** 0.5 + rows) * max(1.0, float(y.abs().max()))
+
+
 @pytest.mark.parametrize("E_bond, n", [(9000, 64), (300, 64), (20000, 128)])
 def test_block_with_both_filter_grids_in_one_launch(pkg, E_bond, n):
     """A block of two graphs against its messages called one by one (a hook that changes nothing keeps a block from handing
