@@ -277,6 +277,14 @@ int mg_tensor_linear_layout(int inds, const float* W, long w_stride_o, long w_st
                             const float* x, long rows, int dim_in, int dim_out,
                             const float* bias, int act, int accumulate,
                             int x_layout, int y_layout, float* y, mg_stream_t stream);
+/* y = x W^T (+ y) for plain rows x_stride floats apart, products and sums in fp32 whatever the linear mode is. */
+int mg_tensor_linear_rows(const float* W, long w_stride_o, long w_stride_i, const float* x, long x_stride, long rows, int dim_in,
+                          int dim_out, int accumulate, float* y, mg_stream_t stream);
+/* y (rows, dim_out) = sum_p x_p W_p^T for x = [x_0 | x_1 | ..] (rows, products dim_in), likewise in fp32, and x_rowmax (rows, products),
+ * the row maxima of |x_p|.  W: host array of at most 8 weights (dim_out, dim_in) of unit column stride; dim_in % 32 == 0, x, the weights
+ * and their rows 16-byte aligned. */
+int mg_tensor_linear_products(const float* const* W, long w_stride_o, int products, const float* x, long rows, int dim_in, int dim_out,
+                              float* y, float* x_rowmax, mg_stream_t stream);
 /* Arithmetic used by the wide plain-row GEMMs (inds = 0 or component-major x, dim_in % 32 == 0):
  *   0  fp32 MFMA (v_mfma_f32_32x32x2_f32);
  *   1  operands split exactly into three bf16 pieces, six bf16 MFMAs per product, fp32
@@ -368,6 +376,8 @@ typedef struct mg_f16x2_linear {
     float* y_rowmax;
 } mg_f16x2_linear;
 int mg_tensor_linear_f16x2_run(const mg_f16x2_linear* args /* host */, mg_stream_t stream);
+/* the same with the rows of x x_stride floats apart (a multiple of 4) */
+int mg_tensor_linear_f16x2_run_strided(const mg_f16x2_linear* args /* host */, long x_stride, mg_stream_t stream);
 int mg_tensor_linear_f16x2_rowmax_parts_sequential(long rows, int dim_in, int dim_out);
 /* Linear, SiLU, Linear, SiLU, Linear (archs/meanflow_painn8.py:38-51) on plain rows as one kernel, the hidden rows staying on
  * chip: x (rows, dim_in) -> y (rows, dim), hidden layers of `dim` columns, packed_W from mg_linear_f16x2_pack_weight, biases

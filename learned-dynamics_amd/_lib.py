@@ -64,6 +64,8 @@ _SIGNATURES = {
     "mg_tensor_linear_wgrad_f16x2_supported": [i64, i32, i32],
     "mg_tensor_linear_wgrad_f16x2_rows": [vp, vp, vp, i64, vp, i64, i64, i64, i32, i32, vp, vp, vp, vp],
     "mg_tensor_linear_wgrad_f16x2": [vp, vp, vp, i64, vp, i64, i64, i32, i32, vp, vp, vp, vp],
+    "mg_tensor_linear_products": [vp, i64, i32, vp, i64, i32, i32, vp, vp, vp],
+    "mg_tensor_linear_rows": [vp, i64, i64, vp, i64, i64, i32, i32, i32, vp, vp],
     "mg_tensor_linear_layout": [i32, vp, i64, i64, vp, i64, i32, i32, vp, i32, i32, i32, i32, vp, vp],
     "mg_bee_edge_geometry": [vp, i64, f32, vp, vp, vp],
     "mg_bee_message": [vp, vp, vp, i32, i64, vp, vp, vp, vp, vp, i32, vp, vp, vp, vp, vp, vp, vp, vp],
@@ -80,6 +82,7 @@ _SIGNATURES = {
     "mg_row_absmax": [vp, i64, i32, vp, vp],
     "mg_linear_f64": [vp, vp, vp, i64, i32, i32, i32, vp, vp],
     "mg_tensor_linear_f16x2_run": [vp, vp],
+    "mg_tensor_linear_f16x2_run_strided": [vp, i64, vp],
     "mg_tensor_linear_f16x2_rowmax_parts_sequential": [i64, i32, i32],
     "mg_linear_f16x2_pack_weight_padded": [vp, i64, i64, i32, i32, i32, vp, vp],
     "mg_linear_f16x2_pack_weights": [vp, i32, vp],

@@ -63,7 +63,7 @@ struct Cfg {
 
 template <int T, int WAVES_M, int WAVES_N, int WM, int WN, bool XVEC, bool SOA_OUT>
 __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N)
-linear_kernel(const float* __restrict__ W, long so, long si, const float* __restrict__ X, long R, int I, int O,
+linear_kernel(const float* __restrict__ W, long so, long si, const float* __restrict__ X, long row_floats, long R, int I, int O,
               const float* __restrict__ bias, int act, int accumulate, float* __restrict__ Y, int out_T) {
     using C = Cfg<T, WAVES_M, WAVES_N, WM, WN>;
     __shared__ float xs[C::RB * C::RS];
@@ -74,7 +74,6 @@ linear_kernel(const float* __restrict__ W, long so, long si, const float* __rest
     const int wave_m = wave / WAVES_N, wave_n = wave % WAVES_N;
     const long r0 = (long)blockIdx.x * C::RB;
     const int n0 = blockIdx.y * C::BN;
-    const long row_floats = (long)I * T;
 
     float16v acc[WM][WN];
 #pragma unroll
@@ -200,25 +199,26 @@ linear_kernel(const float* __restrict__ W, long so, long si, const float* __rest
 
 template <int T, int WAVES_M, int WAVES_N, int WM, int WN>
 int launch_cfg(const float* W, long so, long si, const float* X, long R, int I, int O, const float* bias, int act,
-               int accumulate, float* Y, hipStream_t st, bool soa_out = false, int out_T = 1) {
+               int accumulate, float* Y, hipStream_t st, bool soa_out = false, int out_T = 1, long row_floats = -1) {
+    if (row_floats < 0) row_floats = (long)I * T;
     using C = Cfg<T, WAVES_M, WAVES_N, WM, WN>;
     const long gx = ceil_div(R, C::RB);
     const long gy = ceil_div(O, C::BN);
     MG_REQUIRE(gx <= 0x7fffffffL && gy <= 65535, "mg_tensor_linear: grid too large (rows=%ld dim_out=%d)", R, O);
-    const bool xvec = I > 0 && aligned16(X) && (I % kBK == 0) && (((long)I * T) % 4 == 0);
+    const bool xvec = I > 0 && aligned16(X) && (I % kBK == 0) && (row_floats % 4 == 0);
     dim3 grid((unsigned)gx, (unsigned)gy), block(C::NT);
     if (xvec && soa_out)
         hipLaunchKernelGGL((linear_kernel<T, WAVES_M, WAVES_N, WM, WN, true, true>), grid, block, 0, st, W, so, si, X,
-                           R, I, O, bias, act, accumulate, Y, out_T);
+                           row_floats, R, I, O, bias, act, accumulate, Y, out_T);
     else if (xvec)
         hipLaunchKernelGGL((linear_kernel<T, WAVES_M, WAVES_N, WM, WN, true, false>), grid, block, 0, st, W, so, si, X,
-                           R, I, O, bias, act, accumulate, Y, out_T);
+                           row_floats, R, I, O, bias, act, accumulate, Y, out_T);
     else if (soa_out)
         hipLaunchKernelGGL((linear_kernel<T, WAVES_M, WAVES_N, WM, WN, false, true>), grid, block, 0, st, W, so, si, X,
-                           R, I, O, bias, act, accumulate, Y, out_T);
+                           row_floats, R, I, O, bias, act, accumulate, Y, out_T);
     else
         hipLaunchKernelGGL((linear_kernel<T, WAVES_M, WAVES_N, WM, WN, false, false>), grid, block, 0, st, W, so, si,
-                           X, R, I, O, bias, act, accumulate, Y, out_T);
+                           X, row_floats, R, I, O, bias, act, accumulate, Y, out_T);
     return check_launch("mg_tensor_linear");
 }
 
@@ -239,10 +239,11 @@ int launch_cfg(const float* W, long so, long si, const float* X, long R, int I, 
 //    own L2): x is then fetched from HBM once and re-read from that L2.
 constexpr int kBK1 = 32;
 constexpr int kRS1 = kBK1 + 4;
+constexpr int kMaxProducts = 8;
 
 template <bool WVEC>
 __global__ void __launch_bounds__(256)
-linear_rows_kernel(const float* __restrict__ W, long so, long si, const float* __restrict__ X, long R, int I, int O,
+linear_rows_kernel(const float* __restrict__ W, long so, long si, const float* __restrict__ X, long x_stride, long R, int I, int O,
                    const float* __restrict__ bias, int act, int accumulate, float* __restrict__ Y, int tiles_n,
                    long tiles_total, int out_T) {
     __shared__ __attribute__((aligned(16))) float xs[128 * kRS1];
@@ -279,7 +280,7 @@ linear_rows_kernel(const float* __restrict__ W, long so, long si, const float* _
         for (int j = 0; j < 4; j++) {
             const int r = ld_r + 32 * j;
             float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (r0 + r < R) v = *reinterpret_cast<const float4*>(X + (r0 + r) * I + k0 + ld_c);
+            if (r0 + r < R) v = *reinterpret_cast<const float4*>(X + (r0 + r) * x_stride + k0 + ld_c);
             xv[j] = v;
             float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
             const int n = n0 + r;
@@ -368,7 +369,8 @@ linear_rows_kernel(const float* __restrict__ W, long so, long si, const float* _
 }
 
 int launch_rows(const float* W, long so, long si, const float* X, long R, int I, int O, const float* bias, int act,
-                int accumulate, float* Y, hipStream_t st, int out_T = 1) {
+                int accumulate, float* Y, hipStream_t st, int out_T = 1, long x_stride = -1) {
+    if (x_stride < 0) x_stride = I;
     const long tiles_m = ceil_div(R, 128);
     const int tiles_n = (int)ceil_div(O, 128);
     const long total = tiles_m * tiles_n;
@@ -376,14 +378,152 @@ int launch_rows(const float* W, long so, long si, const float* X, long R, int I,
     MG_REQUIRE(grid <= 0x7fffffffL, "mg_tensor_linear: grid too large (rows=%ld dim_out=%d)", R, O);
     const bool wvec = si == 1 && so % 4 == 0 && aligned16(W);
     if (wvec)
-        hipLaunchKernelGGL(linear_rows_kernel<true>, dim3((unsigned)grid), dim3(256), 0, st, W, so, si, X, R, I, O, bias,
+        hipLaunchKernelGGL(linear_rows_kernel<true>, dim3((unsigned)grid), dim3(256), 0, st, W, so, si, X, x_stride, R, I, O, bias,
                            act, accumulate, Y, tiles_n, total, out_T);
     else
-        hipLaunchKernelGGL(linear_rows_kernel<false>, dim3((unsigned)grid), dim3(256), 0, st, W, so, si, X, R, I, O,
+        hipLaunchKernelGGL(linear_rows_kernel<false>, dim3((unsigned)grid), dim3(256), 0, st, W, so, si, X, x_stride, R, I, O,
                            bias, act, accumulate, Y, tiles_n, total, out_T);
     return check_launch("mg_tensor_linear");
 }
 
+
+// Several linears whose operands lie side by side in rows of x, summed: y = sum_p x[:, p C .. + C] W_p^T, in fp32 throughout and with
+// the row maxima of |x_p| on the way.  A product's sum is a chain of its own, as of one linear after the other.  128 (64) rows a
+// workgroup, slabs of 32 k in two LDS buffers with the loads of the next two in flight; k pairs and strides as in linear_rows_kernel.
+// Five products of 256 channels, us here / in five launches of linear_kernel / bytes at 5 TB/s: 73 728 rows -> 16 109 / 200 / 76,
+// 24 576 -> 64 62 / 165 / 26.  Bound by the slab in turn: with one slab in flight 114 and 98.
+struct ProductWeights { const float* W[kMaxProducts]; };
+template <int WAVES_M, int NI>
+__global__ void __launch_bounds__(256)
+linear_products_kernel(const ProductWeights weights, long so, const float* __restrict__ X, long R, int C, int G, int O,
+                       float* __restrict__ Y, float* __restrict__ xmax, int tiles_n, long tiles_total) {
+    constexpr int WAVES_N = 4 / WAVES_M, TM = 32 * WAVES_M, TN = 32 * NI * WAVES_N, XL = TM / 32, WL = TN / 32;
+    __shared__ __attribute__((aligned(16))) float xs[2][TM * kRS1];
+    __shared__ __attribute__((aligned(16))) float ws[2][TN * kRS1];
+    // XCD-aware tile order
+    const long per_xcd = (tiles_total + 7) / 8, logical = (long)(blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (logical >= tiles_total) return;
+    const long tile_m = logical / tiles_n;
+    const int tile_n = (int)(logical - tile_m * tiles_n);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, khalf = lane >> 5;
+    const int wave_m = wave / WAVES_N, wave_n = wave % WAVES_N;
+    const long r0 = tile_m * TM, row_floats = (long)G * C;
+    const int n0 = tile_n * TN;
+
+    const int ld_r = tid >> 3, ld_c = (tid & 7) * 4;          // + 32 rows per j
+    const float* x_ptr[XL];
+#pragma unroll
+    for (int j = 0; j < XL; j++) {                            // (rows and columns past the end repeat the last one and are not written)
+        const long r = r0 + ld_r + 32 * j;
+        x_ptr[j] = X + (r < R ? r : R - 1) * row_floats + ld_c;
+    }
+    long w_off[WL];
+#pragma unroll
+    for (int j = 0; j < WL; j++) {
+        const int n = n0 + ld_r + 32 * j;
+        w_off[j] = (long)(n < O ? n : O - 1) * so + ld_c;
+    }
+    const int slabs = C / kBK1, total_slabs = G * slabs;
+    struct Slab { float4 x[XL], w[WL]; };
+    int p_load = 0, c_load = 0;                               // the next slab to be requested: slab c_load of product p_load
+    auto load = [&](Slab& v) __attribute__((always_inline)) {
+        const float* W = weights.W[p_load] + c_load * kBK1;
+#pragma unroll
+        for (int j = 0; j < XL; j++) v.x[j] = *reinterpret_cast<const float4*>(x_ptr[j] + (long)p_load * C + c_load * kBK1);
+#pragma unroll
+        for (int j = 0; j < WL; j++) v.w[j] = *reinterpret_cast<const float4*>(W + w_off[j]);
+        // (behind the last slab the same one again, unused: no branch around the loads, which would wait for all of them)
+        const bool next = c_load + 1 == slabs, last = next && p_load + 1 == G;
+        c_load = last ? c_load : (next ? 0 : c_load + 1);
+        p_load += next && !last ? 1 : 0;
+    };
+    float16v acc[NI], sum[NI];
+#pragma unroll
+    for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+        for (int q = 0; q < 16; q++) acc[ni][q] = sum[ni][q] = 0.f;
+    float mx[XL];
+#pragma unroll
+    for (int j = 0; j < XL; j++) mx[j] = 0.f;
+    const int a_off = (wave_m * 32 + (lane & 31)) * kRS1 + khalf * 16, b_off = (wave_n * NI * 32 + (lane & 31)) * kRS1 + khalf * 16;
+
+    int p = 0, c = 0;                                         // the slab to be multiplied
+    auto step = [&](Slab& v, float* xb, float* wb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < XL; j++) {
+            *reinterpret_cast<float4*>(xb + (ld_r + 32 * j) * kRS1 + ld_c) = v.x[j];
+            mx[j] = fmaxf(fmaxf(fmaxf(mx[j], fabsf(v.x[j].x)), fabsf(v.x[j].y)), fmaxf(fabsf(v.x[j].z), fabsf(v.x[j].w)));
+        }
+#pragma unroll
+        for (int j = 0; j < WL; j++) *reinterpret_cast<float4*>(wb + (ld_r + 32 * j) * kRS1 + ld_c) = v.w[j];
+        __syncthreads();                                      // (this buffer is written again behind the next of these)
+        load(v);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+            float a[8], b[NI][8];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const float4 t = *reinterpret_cast<const float4*>(xb + a_off + half * 8 + 4 * k);
+                a[4 * k] = t.x; a[4 * k + 1] = t.y; a[4 * k + 2] = t.z; a[4 * k + 3] = t.w;
+#pragma unroll
+                for (int ni = 0; ni < NI; ni++) {
+                    const float4 u = *reinterpret_cast<const float4*>(wb + b_off + 32 * ni * kRS1 + half * 8 + 4 * k);
+                    b[ni][4 * k] = u.x; b[ni][4 * k + 1] = u.y; b[ni][4 * k + 2] = u.z; b[ni][4 * k + 3] = u.w;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 8; k++)
+#pragma unroll
+                for (int ni = 0; ni < NI; ni++) acc[ni] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[k], b[ni][k], acc[ni], 0, 0, 0);
+        }
+        if (++c < slabs) return;
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+            for (int q = 0; q < 16; q++) { sum[ni][q] += acc[ni][q]; acc[ni][q] = 0.f; }
+#pragma unroll
+        for (int j = 0; j < XL; j++) {
+            float m = mx[j];
+#pragma unroll
+            for (int d = 1; d < 8; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
+            const long r = r0 + ld_r + 32 * j;
+            if ((tid & 7) == 0 && tile_n == 0 && r < R) xmax[r * G + p] = m;
+            mx[j] = 0.f;
+        }
+        c = 0;
+        p++;
+    };
+    Slab even, odd;
+    load(even);
+    load(odd);
+    for (int s = 0; s + 1 < total_slabs; s += 2) {
+        step(even, xs[0], ws[0]);
+        step(odd, xs[1], ws[1]);
+    }
+    if (total_slabs & 1) step(even, xs[0], ws[0]);
+#pragma unroll
+    for (int ni = 0; ni < NI; ni++) {
+        const int n = n0 + (wave_n * NI + ni) * 32 + (lane & 31);
+        if (n >= O) continue;
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            const long r = r0 + wave_m * 32 + 8 * (q / 4) + 4 * khalf + (q % 4);
+            if (r < R) Y[r * O + n] = sum[ni][q];
+        }
+    }
+}
+
+template <int WAVES_M, int NI>
+int launch_products(const ProductWeights& weights, long so, const float* X, long R, int C, int G, int O, float* Y, float* xmax,
+                    hipStream_t st) {
+    const int tiles_n = (int)ceil_div(O, 32 * NI * (4 / WAVES_M));
+    const long total = ceil_div(R, 32 * WAVES_M) * tiles_n, grid = ceil_div(total, 8) * 8;
+    MG_REQUIRE(grid <= 0x7fffffffL, "mg_tensor_linear_products: grid too large (rows=%ld dim_out=%d)", R, O);
+    hipLaunchKernelGGL((linear_products_kernel<WAVES_M, NI>), dim3((unsigned)grid), dim3(256), 0, st, weights, so, X, R, C, G, O, Y, xmax,
+                       tiles_n, total);
+    return check_launch("mg_tensor_linear_products");
+}
 
 // A handful of output channels (readouts: n -> 1 vectors).  The matrix tiles above are 32 columns wide, so a one-column
 // output uses 1/32 of them, and the launch is bound by the latency of its few workgroups' loop over dim_in.  Here a
@@ -599,6 +739,43 @@ int mg_tensor_linear_layout(int inds, const float* W, long w_stride_o, long w_st
     if (cols == 32) return launch_cfg<9, 3, 1, 3, 1>(W, so, si, x, rows, dim_in, dim_out, b, act, accumulate, y, st, soa);
     if (cols == 64) return launch_cfg<9, 3, 1, 3, 2>(W, so, si, x, rows, dim_in, dim_out, b, act, accumulate, y, st, soa);
     return launch_cfg<9, 3, 2, 3, 2>(W, so, si, x, rows, dim_in, dim_out, b, act, accumulate, y, st, soa);
+}
+
+int mg_tensor_linear_rows(const float* W, long w_stride_o, long w_stride_i, const float* x, long x_stride, long rows, int dim_in,
+                          int dim_out, int accumulate, float* y, mg_stream_t stream) {
+    MG_REQUIRE(rows >= 0 && dim_in >= 0 && dim_out >= 0 && x_stride >= dim_in, "mg_tensor_linear_rows: bad size");
+    if (rows == 0 || dim_out == 0) return MG_OK;
+    MG_REQUIRE(y != nullptr && (dim_in == 0 || (W != nullptr && x != nullptr)), "mg_tensor_linear_rows: null pointer");
+    hipStream_t st = (hipStream_t)stream;
+    const long so = w_stride_o, si = w_stride_i;
+    if (x_stride == dim_in) {
+        if (dim_out <= 4 && dim_in >= 16 && dim_in % 4 == 0 && aligned16(x))
+            return launch_few_outputs<1>(W, so, si, x, rows, dim_in, dim_out, nullptr, 0, accumulate, 0, y, st);
+        if (dim_in >= 1 && dim_in <= few_inputs_max(1))
+            return launch_few_inputs<1>(W, so, si, x, rows, dim_in, dim_out, nullptr, 0, accumulate, 0, y, st);
+    }
+    if (dim_out > 64 && dim_in % kBK1 == 0 && x_stride % 4 == 0 && aligned16(x))
+        return launch_rows(W, so, si, x, rows, dim_in, dim_out, nullptr, 0, accumulate, y, st, 1, x_stride);
+    if (dim_out <= 32) return launch_cfg<1, 4, 1, 2, 1>(W, so, si, x, rows, dim_in, dim_out, nullptr, 0, accumulate, y, st, false, 1, x_stride);
+    if (dim_out <= 64) return launch_cfg<1, 2, 2, 2, 1>(W, so, si, x, rows, dim_in, dim_out, nullptr, 0, accumulate, y, st, false, 1, x_stride);
+    return launch_cfg<1, 2, 2, 2, 2>(W, so, si, x, rows, dim_in, dim_out, nullptr, 0, accumulate, y, st, false, 1, x_stride);
+}
+
+int mg_tensor_linear_products(const float* const* W, long w_stride_o, int products, const float* x, long rows, int dim_in, int dim_out,
+                              float* y, float* x_rowmax, mg_stream_t stream) {
+    MG_REQUIRE(W && products >= 1 && products <= kMaxProducts && rows >= 0 && dim_in > 0 && dim_in % kBK1 == 0 && dim_out >= 0,
+               "mg_tensor_linear_products: 1 to %d weights, dim_in a multiple of %d", kMaxProducts, kBK1);
+    if (rows == 0 || dim_out == 0) return MG_OK;
+    MG_REQUIRE(x && y && x_rowmax && aligned16(x) && w_stride_o % 4 == 0, "mg_tensor_linear_products: null or unaligned pointer");
+    ProductWeights weights{};
+    for (int p = 0; p < products; p++) {
+        MG_REQUIRE(W[p] && aligned16(W[p]), "mg_tensor_linear_products: null or unaligned weight");
+        weights.W[p] = W[p];
+    }
+    hipStream_t st = (hipStream_t)stream;
+    if (dim_out <= 32) return launch_products<4, 1>(weights, w_stride_o, x, rows, dim_in, products, dim_out, y, x_rowmax, st);
+    if (dim_out <= 64) return launch_products<2, 1>(weights, w_stride_o, x, rows, dim_in, products, dim_out, y, x_rowmax, st);
+    return launch_products<2, 2>(weights, w_stride_o, x, rows, dim_in, products, dim_out, y, x_rowmax, st);
 }
 
 int mg_set_linear_mode(int mode) {

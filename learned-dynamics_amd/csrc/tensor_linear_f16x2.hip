@@ -219,7 +219,7 @@ constexpr int streaming_waves(int waves, int ni) { return waves == 4 && ni <= 2 
 // three times (apart_of)
 template <int WAVES, int NI, bool APART>
 __global__ void __launch_bounds__(64 * WAVES, APART ? 1 : streaming_waves(WAVES, NI))
-linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restrict__ w_inv, const float* __restrict__ X,
+linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restrict__ w_inv, const float* __restrict__ X, long x_stride,
                          const float* __restrict__ xmax, int xmax_parts, long xmax_stride, long xmax_div, long R, int I,
                          int O, int O_pad, const float* __restrict__ bias, int act, int accumulate,
                          float* __restrict__ Y, float* __restrict__ ymax, int tiles_n, long tiles_total, int out_T,
@@ -261,7 +261,7 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
     // this lane's row of x (clamped past the end: those accumulators are never written)
     const long my_row = r0 + wave * 32 + m;
     const long ld_row = my_row < R ? my_row : R - 1;
-    const float* xrow = X + ld_row * I + 16 * g;
+    const float* xrow = X + ld_row * x_stride + 16 * g;
     float sx;
     bool odd;                                                // this wave has rows (columns: below) that the pieces cannot carry
     {
@@ -521,7 +521,7 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
             const float isx = inv_sx[rl], iw = w_inv[n];
             if (isx == isx && iw == iw) continue;
             const long row = r / out_T, addr = (row * O + n) * out_T + (r - row * out_T);
-            const float v = activate(row_in_fp32(X + r * I, Wp, plane_elems, n, I, iw) + (bias && r < bias_rows ? bias[n] : 0.f), act);
+            const float v = activate(row_in_fp32(X + r * x_stride, Wp, plane_elems, n, I, iw) + (bias && r < bias_rows ? bias[n] : 0.f), act);
             Y[addr] = accumulate ? v + Y[addr] : v;
         }
     }
@@ -547,7 +547,7 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
 template <int WAVES, int NI>
 __global__ void __launch_bounds__(64 * WAVES)
 linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restrict__ w_inv,
-                                const float* __restrict__ X, const float* __restrict__ xmax, int xmax_parts,
+                                const float* __restrict__ X, long x_stride, const float* __restrict__ xmax, int xmax_parts,
                                 long xmax_stride, long xmax_div, long R, int I, int O, int O_pad,
                                 const float* __restrict__ bias, int act, int accumulate, float* __restrict__ Y,
                                 float* __restrict__ ymax, int tiles_n, int out_T, float bound_mul, float bound_add,
@@ -568,7 +568,7 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
 
     const long my_row = r0 + m;
     const long ld_row = my_row < R ? my_row : R - 1;
-    const float* xrow = X + ld_row * I + 16 * g;
+    const float* xrow = X + ld_row * x_stride + 16 * g;
     float sx;
     {
         float amax = 0.f;
@@ -685,7 +685,7 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
             const float isx = inv_sx[rl], iw = w_inv[n];
             if (isx == isx && iw == iw) continue;
             const long row = r / out_T, addr = (row * O + n) * out_T + (r - row * out_T);
-            const float v = activate(row_in_fp32(X + r * I, Wp, plane_elems, n, I, iw) + (bias && r < bias_rows ? bias[n] : 0.f), act);
+            const float v = activate(row_in_fp32(X + r * x_stride, Wp, plane_elems, n, I, iw) + (bias && r < bias_rows ? bias[n] : 0.f), act);
             Y[addr] = accumulate ? v + Y[addr] : v;
         }
     }
@@ -748,7 +748,7 @@ inline Shape choose_shape(long R, int I, int O) {
 }
 
 // A reduction of more than 512 in tiles of at most 128 columns keeps the small products apart, in a second set of accumulators.
-// The five rank-1 or rank-2 products of the message layers side by side, K = 1280, against float64: 2.7e-7 of the
+// K = 1280 (the five rank-1 or rank-2 products of a layer side by side, in inference) against float64: 2.7e-7 of the
 // result's 2-norm; in one accumulator 4.3e-7, five linears of K = 256 and a sum 3.5e-7, in fp32 6.5e-7.  Sequential
 // reductions take such a tile for every width; others keep the 256-column tile, which has no registers for the second set.
 inline bool apart_of(int I, int ni) { return I > 512 && ni <= 4; }
@@ -759,7 +759,7 @@ inline Shape choose_sequential(long R, int I, int O) {
 }
 
 template <int WAVES, int NI, bool APART = false>
-int launch(const _Float16* planes, const float* w_inv, const float* x, const float* xmax, int parts, long stride,
+int launch(const _Float16* planes, const float* w_inv, const float* x, long x_stride, const float* xmax, int parts, long stride,
            long div, long rows, int I, int O, int O_pad, const float* bias, int act, int accumulate, float* y,
            float* ymax, int out_T, float bound_mul, float bound_add, long bias_rows, hipStream_t st) {
     const long tiles_m = ceil_div(rows, 32 * WAVES);
@@ -768,7 +768,7 @@ int launch(const _Float16* planes, const float* w_inv, const float* x, const flo
     const long grid = ceil_div(total, 8) * 8;
     MG_REQUIRE(grid <= 0x7fffffffL, "mg_tensor_linear_f16x2: grid too large (rows=%ld dim_out=%d)", rows, O);
     hipLaunchKernelGGL((linear_rows_f16x2_kernel<WAVES, NI, APART>), dim3((unsigned)grid), dim3(64 * WAVES), 0, st, planes,
-                       w_inv, x, xmax, parts, stride, div, rows, I, O, O_pad, bias, act, accumulate, y, ymax, tiles_n,
+                       w_inv, x, x_stride, xmax, parts, stride, div, rows, I, O, O_pad, bias, act, accumulate, y, ymax, tiles_n,
                        total, out_T, bound_mul, bound_add, bias_rows);
     return check_launch("mg_tensor_linear_f16x2");
 }
@@ -886,7 +886,13 @@ int mg_tensor_linear_f16x2_scaled_bound(const void* packed_W, const float* x, co
 
 int mg_tensor_linear_f16x2_run(const mg_f16x2_linear* args, mg_stream_t stream) {
     MG_REQUIRE(args != nullptr, "mg_tensor_linear_f16x2: null pointer");
+    return mg_tensor_linear_f16x2_run_strided(args, args->dim_in, stream);
+}
+
+int mg_tensor_linear_f16x2_run_strided(const mg_f16x2_linear* args, long x_stride, mg_stream_t stream) {
+    MG_REQUIRE(args != nullptr, "mg_tensor_linear_f16x2: null pointer");
     const mg_f16x2_linear& a = *args;
+    MG_REQUIRE(x_stride >= a.dim_in && x_stride % 4 == 0, "mg_tensor_linear_f16x2: x_stride must be a multiple of 4, at least dim_in");
     MG_REQUIRE(a.bound_mul >= 0.f && a.bound_add >= 0.f && a.bound_mul == a.bound_mul && a.bound_add == a.bound_add,
                "mg_tensor_linear_f16x2: the bound's factor and offset must be non-negative numbers");
     MG_REQUIRE(a.rows >= 0 && a.dim_in > 0 && a.dim_out >= 0, "mg_tensor_linear_f16x2: bad size");
@@ -915,7 +921,7 @@ int mg_tensor_linear_f16x2_run(const mg_f16x2_linear* args, mg_stream_t stream) 
 #define MG_SPLITK(WV, N)                                                                                                   \
     if (sk.waves == WV && sk.ni == N)                                                                                      \
         hipLaunchKernelGGL((linear_rows_splitk_f16x2_kernel<WV, N>), dim3((unsigned)tiles), dim3(64 * WV), 0, st, planes,  \
-                           w_inv, a.x, a.x_rowmax, a.x_rowmax_parts, a.x_rowmax_stride, a.x_rows_per_bound, a.rows,        \
+                           w_inv, a.x, x_stride, a.x_rowmax, a.x_rowmax_parts, a.x_rowmax_stride, a.x_rows_per_bound, a.rows, \
                            a.dim_in, a.dim_out, O_pad, a.bias, a.act, a.accumulate, a.y, a.y_rowmax, tiles_n, a.out_comps, \
                            a.bound_mul, a.bound_add, a.bias_rows)
         MG_SPLITK(8, 1);
@@ -930,7 +936,7 @@ int mg_tensor_linear_f16x2_run(const mg_f16x2_linear* args, mg_stream_t stream) 
     // 73 728 rows 40 against 65); longer reductions keep the tile that re-reads x least
     if (a.out_comps == 9 && a.dim_in <= 64 && a.dim_out % 64 == 0 && a.act == 0 && a.bias == nullptr) sh = Shape{2, 4};
 #define MG_F16X2_LAUNCH(WV, ...)                                                                                           \
-    return launch<WV, __VA_ARGS__>(planes, w_inv, a.x, a.x_rowmax, a.x_rowmax_parts, a.x_rowmax_stride, a.x_rows_per_bound, a.rows, \
+    return launch<WV, __VA_ARGS__>(planes, w_inv, a.x, x_stride, a.x_rowmax, a.x_rowmax_parts, a.x_rowmax_stride, a.x_rows_per_bound, a.rows, \
                          a.dim_in, a.dim_out, O_pad, a.bias, a.act, a.accumulate, a.y, a.y_rowmax, a.out_comps,            \
                          a.bound_mul, a.bound_add, a.bias_rows, st)
     if (apart_of(a.dim_in, sh.ni)) {

@@ -226,14 +226,14 @@ int64_t rowmax_parts(int64_t rows, int64_t dim_in, int64_t dim_out, bool sequent
 // x (rows, k) plain rows; y preallocated; packed: W's planes where the caller holds them
 void run_f16x2(const at::Tensor& W, int64_t k, const float* x, int64_t rows, const Bound& b, const OptTensor& bias, int act,
                bool accumulate, int out_comps, at::Tensor& y, at::Tensor* ymax, bool sequential, int64_t bias_rows = -1,
-               const OptTensor& packed = OptTensor()) {
+               const OptTensor& packed = OptTensor(), int64_t x_stride = -1, int64_t max_column = 0) {
     const at::Tensor planes = packed.has_value() ? *packed : packed_f16x2(W, k);
     const at::Tensor& base = *b.base;
     mg_f16x2_linear a{};
     a.packed_W = planes.data_ptr();
     a.x = x;
-    a.x_rowmax = fp(base);
-    a.x_rowmax_parts = (int)base.size(1);
+    a.x_rowmax = fp(base) + max_column;                        // (x_stride: a column of `base` for each block of columns of x)
+    a.x_rowmax_parts = x_stride < 0 ? (int)base.size(1) : 1;
     a.x_rowmax_stride = base.size(0) > 1 || rows == b.rows_per ? base.size(1) : 0;
     a.x_rows_per_bound = b.rows_per;
     a.bound_mul = b.mul;
@@ -249,7 +249,7 @@ void run_f16x2(const at::Tensor& W, int64_t k, const float* x, int64_t rows, con
     a.sequential = sequential;
     a.y = fp(y);
     a.y_rowmax = ymax ? fp(*ymax) : nullptr;
-    check(mg_tensor_linear_f16x2_run(&a, stream_of(y)));
+    check(mg_tensor_linear_f16x2_run_strided(&a, x_stride < 0 ? k : x_stride, stream_of(y)));
 }
 
 void check_bound(const at::Tensor& b, int64_t rows, int64_t rows_per) {
@@ -821,6 +821,84 @@ std::vector<OptTensor> pack_ahead(const Tensors& weights, const Tensors& passing
     for (size_t k = 0, at = kept; k < passing.size(); k++)
         if (packs_f16x2(passing[k])) out[k] = planes[at++];
     return out;
+}
+
+// sum_k W_k x_k for x = [x_1 | x_2 | ..] (R, G C), one plain row per (row, component) of tensors of T components: the arithmetic of
+// tensor linears one by one (linear_fwd), each x_k with row maxima, and each weight with scales, of its own.  Also
+// the row maxima (R, G) of |x_k| where they were needed.
+std::tuple<at::Tensor, OptTensor> row_linears_fwd(const at::Tensor& x, const Tensors& W, int64_t T, bool sequential) {
+    check_input(x, "x");
+    TORCH_CHECK(!W.empty() && (T == 1 || T == 3 || T == 9) && x.dim() == 2, "row_linears: operands");
+    const int64_t R = x.size(0), G = (int64_t)W.size(), O = W[0].size(0), C = W[0].size(1);
+    for (const at::Tensor& w : W)
+        TORCH_CHECK(w.is_cuda() && w.scalar_type() == at::kFloat && w.dim() == 2 && w.size(0) == O && w.size(1) == C && x.size(1) == G * C,
+                    "row_linears: weights (dim_out, chan), x (rows, weights chan)");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    at::Tensor y = floats(x, {R, O});
+    const bool split = mg_get_linear_mode() == kModeF16x2 && f16x2_takes(R, C, O, x) &&
+                       (T == 1 ? !sequential || R >= 256 : component_rows_take(R, C, O, sequential));
+    OptTensor x_max;
+    if (split) {
+        pack_ahead(W);
+        x_max = row_absmax(x.view({R * G, C})).view({R, G});
+    }
+    std::vector<const float*> weights;
+    for (const at::Tensor& w : W)
+        if (w.stride(1) == 1 && w.stride(0) == W[0].stride(0) && w.stride(0) % 4 == 0 && aligned16(w)) weights.push_back(fp(w));
+    if (!split && G <= 8 && C % 32 == 0 && aligned16(x) && (int64_t)weights.size() == G) {
+        at::Tensor m = floats(x, {R, G});
+        check(mg_tensor_linear_products(weights.data(), W[0].stride(0), (int)G, fp(x), R, (int)C, (int)O, fp(y), fp(m), stream_of(x)));
+        return {y, m};
+    }
+    for (int64_t k = 0; k < G; k++) {
+        if (split)
+            run_f16x2(W[k], C, fp(x) + k * C, R, Bound{x_max}, OptTensor(), kActNone, k > 0, 1, y, nullptr, sequential, -1, OptTensor(),
+                      G * C, k);
+        else
+            check(mg_tensor_linear_rows(fp(W[k]), W[k].stride(0), W[k].stride(1), fp(x) + k * C, G * C, R, (int)C, (int)O, k > 0, fp(y),
+                                        stream_of(x)));
+    }
+    return {y, x_max};
+}
+
+// Its gradients for x and the weights, (dim_out, chan) each
+std::tuple<OptTensor, Tensors> row_linears_bwd(const at::Tensor& dy, const at::Tensor& x, const Tensors& W, OptTensor x_max, int64_t T,
+                                               bool want_x, bool want_W) {
+    check_input(dy, "dy");
+    check_input(x, "x");
+    const int64_t R = x.size(0), G = (int64_t)W.size(), O = W[0].size(0), C = W[0].size(1);
+    TORCH_CHECK(dy.dim() == 2 && dy.size(0) == R && dy.size(1) == O && x.size(1) == G * C, "row_linears: gradient sizes");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    const bool f16x2 = mg_get_linear_mode() == kModeF16x2;
+    const bool split_x = f16x2 && f16x2_takes(R, O, G * C, dy) && (T == 1 || component_rows_take(R, O, C, false));
+    const bool split_W = f16x2 && aligned16(x) && aligned16(dy) && (T == 1 || std::max(C, O) <= 256) &&
+                         mg_tensor_linear_wgrad_f16x2_supported(R, (int)(G * C), (int)O);
+    OptTensor dx, dy_max;
+    if ((want_x && split_x) || (want_W && split_W)) dy_max = row_absmax(dy);
+    if (want_x) {
+        // (one linear: the columns' scales are those of the transposed weights' rows, one for each channel of each x_k)
+        const at::Tensor Wt = (G == 1 ? W[0] : at::cat(W, 1)).t();
+        dx = floats(x, x.sizes());
+        if (split_x) run_f16x2(Wt, O, fp(dy), R, Bound{dy_max}, OptTensor(), kActNone, false, 1, *dx, nullptr, false, -1,
+                               G == 1 ? OptTensor() : pack_ahead({}, {Wt})[0]);
+        else check(mg_tensor_linear_rows(fp(Wt), Wt.stride(0), Wt.stride(1), fp(dy), O, R, (int)O, (int)(G * C), 0, fp(*dx), stream_of(x)));
+    }
+    Tensors dW;
+    if (want_W) {
+        at::Tensor all = floats(x, {O, G * C});
+        size_t n = 0;
+        check(mg_tensor_linear_wgrad_workspace_bytes(R, (int)(G * C), (int)O, &n));
+        at::Tensor ws = bytes_like(x, n);
+        if (split_W) {
+            if (!x_max.has_value()) x_max = row_absmax(x.view({R * G, C}));
+            check(mg_tensor_linear_wgrad_f16x2(fp(dy), fp(x), fp(dy_max), R, fp(x_max), R * G, R, (int)(G * C), (int)O, ws.data_ptr(),
+                                               fp(all), nullptr, stream_of(x)));
+        } else {
+            check(mg_tensor_linear_wgrad(0, fp(dy), fp(x), R, (int)(G * C), (int)O, ws.data_ptr(), fp(all), stream_of(x)));
+        }
+        for (int64_t k = 0; k < G; k++) dW.push_back(all.narrow(1, k * C, C));
+    }
+    return {dx, dW};
 }
 
 // y = x W^T, with the bias added to the first bias_rows rows
@@ -1467,6 +1545,8 @@ void register_ops(pybind11::module_& m) {
     m.def("linear_fwd", &linear_fwd);
     m.def("component_rows_take", &component_rows_take);
     m.def("linear_wgrad", &linear_wgrad);
+    m.def("row_linears_fwd", &row_linears_fwd);
+    m.def("row_linears_bwd", &row_linears_bwd);
     m.def("silu_order", &silu_order);
     m.def("linear_chain", &linear_chain);
     m.def("filter_grid", &filter_grid);

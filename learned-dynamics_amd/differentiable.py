@@ -972,8 +972,7 @@ def _as_rows(P0, S1, S2):
 class _MessageProducts(torch.autograd.Function):
     """The same with everything between the node operands and the per-node sums folded into kernels.  by_label: operands
     and 13 results as in the plain formulation; else v_node (nodes, 3, chan), d_node (nodes, 9, chan) and the results as the plain
-    rows of P0, S1, S2 (ops.bee_message), which the output linears of a rank read as one, and then bounds of the row maxima of
-    |S1|, |S2| per node and of |P0| (empty when not known).
+    rows of P0, S1, S2 (ops.bee_message), which the output linears of a rank read side by side.
     Forward: the inference kernel of the layer (mg_bee_message: filters formed in registers, node rows gathered at the destination,
     products summed over the edges of a node; only the three scalar products are stored per edge) when `enc_source`
     = (the 8 radial functions, weight and bias of the encoding linear) is given, else the indexed product kernel and
@@ -990,15 +989,13 @@ class _MessageProducts(torch.autograd.Function):
         ctx.save_for_forward(a_node, v_node, d_node, enc, rh)
         N, C = a_node.shape
         left = a_node, v_node, d_node
-        node_max = edge_max = enc.new_empty(0)
         if enc_source is not None:
             enc8, W, b = enc_source
             b = b if b is not None else torch.zeros(C, dtype=torch.float32, device=enc.device)
             operands = by_src.row_ptr, by_dst.index, rh, enc8.contiguous(), *(_by_component(*left) if by_label else left)
-            weights = W.detach().contiguous(), b.detach().contiguous()
+            stacked = ops.bee_message(*operands, W.detach().contiguous(), b.detach().contiguous())
             if by_label:
-                return ops.unstack_products(*ops.bee_message(*operands, *weights))
-            *stacked, node_max, edge_max = ops.bee_message(*operands, *weights, want_node_max=True)
+                return ops.unstack_products(*stacked)
         else:
             phi_v, phi_d = ops.bee_edge_filters_fwd(enc, rh)
             prods = ops.bee_fwd_indexed(*(left if by_label else (t.contiguous() for t in _by_channel(*left))), by_dst.index, enc,
@@ -1008,8 +1005,7 @@ class _MessageProducts(torch.autograd.Function):
             if by_label:
                 return prods
             stacked = ops.stack_products(prods)
-        ctx.mark_non_differentiable(node_max, edge_max)
-        return (*_as_rows(*stacked), node_max, edge_max)
+        return _as_rows(*stacked)
 
     @staticmethod
     def jvp(ctx, a_t, v_t, d_t, enc_t, rh_t, *_):
@@ -1026,7 +1022,7 @@ class _MessageProducts(torch.autograd.Function):
         prods = [a + b for a, b in zip(Bee.apply(*gather(left_t), enc, phi_v, phi_d),
                                        Bee.apply(*gather(left), enc_t.contiguous(), phi_v_t.contiguous(), phi_d_t.contiguous()))]
         prods = tuple(p if lab[2] == "0" else gl._ScatterSum.apply(p.contiguous(), by_src) for lab, p in zip(ops.BEE_ORDER, prods))
-        return prods if by_label else (*_as_rows(*ops.stack_products(prods)), None, None)
+        return prods if by_label else _as_rows(*ops.stack_products(prods))
 
     @staticmethod
     def backward(ctx, *dys):
@@ -1054,8 +1050,8 @@ class _MessageProducts(torch.autograd.Function):
 
 class _NodeProducts(torch.autograd.Function):
     """The 13 products of operands (rows, chan), (rows, 3, chan), (rows, 9, chan) as the plain rows of P0, P1, P2
-    (ops.bee_node_products), and bounds of the row maxima of all of them per row (empty when not known).  A recorded backward
-    pass differentiates the product function instead, forward mode is the product rule."""
+    (ops.bee_node_products).  A recorded backward pass differentiates the product function instead, forward mode is the
+    product rule."""
 
     @staticmethod
     def forward(ctx, *operands):
@@ -1063,17 +1059,14 @@ class _NodeProducts(torch.autograd.Function):
         ctx.save_for_backward(*operands)
         ctx.save_for_forward(*operands)
         ctx.set_materialize_grads(False)
-        *stacked, node_max = ops.bee_node_products(*operands, want_node_max=True)
-        node_max = node_max if node_max is not None else operands[0].new_empty(0)
-        ctx.mark_non_differentiable(node_max)
-        return (*_as_rows(*stacked), node_max)
+        return _as_rows(*ops.bee_node_products(*operands))
 
     @staticmethod
     def jvp(ctx, *tangents):
         operands = ctx.saved_tensors
         tangents = [torch.zeros_like(x) if t is None else t for t, x in zip(tangents, operands)]
         left, right = _NodeProducts.apply(*tangents[:3], *operands[3:]), _NodeProducts.apply(*operands[:3], *tangents[3:])
-        return (*(a + b for a, b in zip(left[:3], right[:3])), None)
+        return tuple(a + b for a, b in zip(left, right))
 
     @staticmethod
     def backward(ctx, *dys):
@@ -1097,22 +1090,67 @@ def _component_rows(x):
     return x.flatten(2).transpose(1, 2).reshape(-1, x.shape[1])
 
 
+def _rows_of_rank(x, rank):
+    """(rows, chan, 3, ..) from plain rows (rows 3^rank, chan)"""
+    return x if rank == 0 else x.reshape(-1, 3 ** rank, x.shape[-1]).transpose(1, 2).reshape(-1, x.shape[-1], *[3] * rank)
+
+
+class _RowLinears(torch.autograd.Function):
+    """sum_k W_k x_k for x = [x_1 | x_2 | ..] on plain rows, one per (row, component) of tensors of a rank: tensor linears that
+    lie side by side.  The arithmetic, its fp32 line included, is that of one linear after the other (see _TensorLinearFn): the
+    x_k may differ in magnitude by any factor, so each has scales of its own."""
+
+    @staticmethod
+    def forward(ctx, rank, sequential, x, *W):
+        x = x.contiguous()
+        y, x_max = ops.row_linears_fwd(x, W, 3 ** rank, sequential)
+        ctx.rank = rank
+        ctx.save_for_backward(x, x_max, *W)
+        ctx.save_for_forward(x, x_max, *W)
+        ctx.set_materialize_grads(False)
+        return y
+
+    @staticmethod
+    def jvp(ctx, _rank, _sequential, x_t, *W_t):
+        x, _, *W = ctx.saved_tensors
+        parts = [] if x_t is None else [_RowLinears.apply(ctx.rank, False, x_t, *W)]
+        if any(t is not None for t in W_t):
+            parts.append(_RowLinears.apply(ctx.rank, False, x, *(torch.zeros_like(w) if t is None else t for w, t in zip(W, W_t))))
+        return sum(parts[1:], parts[0]) if parts else None
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, x_max, *W = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        if dy is None:
+            return (None,) * len(need)
+        if torch.is_grad_enabled():
+            return (None, None) + _recorded_gradients(lambda x, *W: (_row_linears_plain(ctx.rank, x, W),), (x, *W), need[2:], (dy,))
+        dy = dy.contiguous()
+        dx, dW = ops.row_linears_bwd(dy, x, W, x_max, 3 ** ctx.rank, need[2], any(need[3:]))
+        return (None, None, dx) + tuple(d if nd else None for d, nd in zip(dW or [None] * len(W), need[3:]))
+
+
+def _row_linears_plain(rank, x, W):
+    """The same as linears one after the other."""
+    y = [tensor_linear(rank, w, _rows_of_rank(x_k, rank)) for w, x_k in zip(W, x.split(W[0].shape[1], dim=1))]
+    y = sum(y[1:], y[0])
+    return y if rank == 0 else _component_rows(y)
+
+
 def _linear_by_component(lin, rank, rows):
     """A TensLinear of rank 0, 1 or 2 on the plain rows of x -> (rows of x, chan) or (rows of x, 3^rank, chan)."""
-    y = tensor_linear(0, lin.W, rows, sequential=torch.is_grad_enabled())
-    return y if rank == 0 else y.reshape(-1, 3 ** rank, y.shape[-1])
+    if rank == 0:
+        return tensor_linear(0, lin.W, rows, sequential=torch.is_grad_enabled())
+    y = _RowLinears.apply(rank, torch.is_grad_enabled(), rows, lin.W)
+    return y.reshape(-1, 3 ** rank, y.shape[-1])
 
 
-def _linears_of_rank(mod, rank, P, bound, rows):
-    """The output linears of one rank, summed: one linear on the plain rows P, whose weights lie side by side.  Returns
-    (rows, dim), (rows, dim, 3) or (rows, dim, 3, 3)."""
-    W = torch.cat([getattr(mod, f"Y_{lab}").W for lab in ops.STACKED[rank]], dim=1)
-    if not bound.numel():
-        bound = None
-    elif rank:
-        bound = bound.repeat_interleave(3 ** rank, dim=0)
-    y = tensor_linear(0, W, P, x_bound=bound, sequential=torch.is_grad_enabled())
-    return y if rank == 0 else y.reshape(rows, 3 ** rank, -1).transpose(1, 2).reshape(rows, -1, *[3] * rank)
+def _linears_of_rank(mod, rank, P):
+    """The output linears of one rank on the plain rows P of their products, summed: (rows, dim), (rows, dim, 3) or
+    (rows, dim, 3, 3)."""
+    return _rows_of_rank(_RowLinears.apply(rank, torch.is_grad_enabled(), P, *(getattr(mod, f"Y_{lab}").W for lab in ops.STACKED[rank])),
+                         rank)
 
 
 def _plain_linears(mod, operands):
@@ -1184,10 +1222,9 @@ def bee_messages(msg, graph, r_ij, x_a, x_v, x_d):
         a, v, d = (gl._flat_nodes(graph, t) for t in (x_a, x_v, x_d))
         nodes = [_linear_by_component(lin, k, x)
                  for k, (lin, x) in enumerate(zip((msg.L0, msg.L1, msg.L2), (a, _component_rows(v), _component_rows(d))))]
-        P0, S1, S2, node_max, edge_max = _MessageProducts.apply(*nodes, enc, rh, graph.by_dst, graph.by_src,
-                                                                (enc8.detach(), msg.lin_enc.weight, msg.lin_enc.bias), False)
-        psi_a = _linears_of_rank(msg, 0, P0, edge_max, None)
-        sums = [_linears_of_rank(msg, k, S, node_max, B * N) for k, S in ((1, S1), (2, S2))]
+        P0, S1, S2 = _MessageProducts.apply(*nodes, enc, rh, graph.by_dst, graph.by_src,
+                                            (enc8.detach(), msg.lin_enc.weight, msg.lin_enc.bias), False)
+        psi_a, *sums = (_linears_of_rank(msg, k, P) for k, P in enumerate((P0, S1, S2)))
         psi_a = psi_a + mlp_leaky(msg.mlp_a, psi_a)
         return (mul(gl.edges_reduce_src(graph, psi_a), 0.1), *(mul(t.reshape(B, N, *t.shape[1:]), 0.1) for t in sums))
     prods = message_products(graph, msg.L0(x_a), msg.L1(x_v), msg.L2(x_d), enc, rh,
@@ -1226,8 +1263,7 @@ def self_tens_prods(mod, x_a, x_v, x_d):
         rows = a, _component_rows(v), _component_rows(d)
         operands = [_linear_by_component(lin, k, x) for side in ((mod.L0, mod.L1, mod.L2), (mod.R0, mod.R1, mod.R2))
                     for k, (lin, x) in enumerate(zip(side, rows))]
-        *stacked, node_max = _NodeProducts.apply(*operands)
-        y_a, y_v, y_d = (_linears_of_rank(mod, k, P, node_max, a.shape[0]) for k, P in enumerate(stacked))
+        y_a, y_v, y_d = (_linears_of_rank(mod, k, P) for k, P in enumerate(_NodeProducts.apply(*operands)))
     else:
         prods = Bee.apply(mod.L0(a), mod.L1(v), mod.L2(d), mod.R0(a), mod.R1(v), mod.R2(d))
         y_a, y_v, y_d = apply_tens_prod_submodules(mod, prods)

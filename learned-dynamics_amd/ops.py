@@ -1229,6 +1229,7 @@ def tensor_linear_wgrad(inds, dy, x, dy_bound=None, x_bound=None, want_bias=Fals
 
 
 # ------------------------------------------------- PaiNN layers under differentiation (values, or values and tangents)
+row_linears_fwd, row_linears_bwd = _ext.row_linears_fwd, _ext.row_linears_bwd
 mlp_silu_fwd = _ext.mlp_silu_fwd
 mlp_silu_bwd = _ext.mlp_silu_bwd
 mlp_leaky_takes, mlp_leaky_fwd, mlp_leaky_bwd = _ext.mlp_leaky_takes, _ext.mlp_leaky_fwd, _ext.mlp_leaky_bwd

@@ -1263,6 +1263,57 @@ def test_rank012_layers_on_stacked_products(pkg, chan, dims, N, E):
                 assert float((x - y).abs().max()) <= 1e-5 * max(float(y.abs().max()), 1e-3), (type(module).__name__, k)
 
 
+def _by_rank(x, rank):
+    return x if rank == 0 else x.reshape(-1, 3 ** rank, x.shape[1]).transpose(1, 2).reshape(-1, x.shape[1], *[3] * rank).contiguous()
+
+
+@pytest.mark.parametrize("rank, C, O, N", [(0, 256, 64, 100), (0, 256, 256, 5000), (0, 192, 5, 4100), (1, 256, 64, 100), (1, 192, 64, 1500),
+                                           (1, 256, 96, 11000), (2, 256, 16, 500), (2, 256, 64, 3700), (2, 24, 3, 600), (2, 512, 64, 500)])
+def test_linears_side_by_side_of_any_magnitude(pkg, ops, rank, C, O, N):
+    """Tensor linears whose operands lie side by side, each 1e-3 to 1e-8 as large as the first, forward and in the gradient of
+    the operands, against float64 and against the linears one after the other.  Tolerance: pieces of 22 bits
+    of the largest of a row (of a weight, of a gradient) leave 2^-22 of it per term, 2^-21 in a product of two, and the terms' errors
+    are as independent as the terms: 2^-21 of the 2-norm; sums in fp32 in chains of K = C add 2^-24 sqrt(K)."""
+    diff = importlib.import_module("learned-dynamics_amd.differentiable")
+    g = torch.Generator().manual_seed(N)
+    sizes = (1.0, 1e-3, 1e-8) if rank == 0 else (1.0, 1e-3, 1e-5, 1e-6, 1e-8)
+    R, G = N * 3 ** rank, len(sizes)
+    x = torch.cat([m * torch.randn(R, C, generator=g) for m in sizes], dim=1).cuda()
+    W = [torch.randn(O, C, generator=g).cuda().requires_grad_() for _ in sizes]
+    dy = torch.randn(R, O, generator=g).cuda()
+    x.requires_grad_()
+    y = diff._RowLinears.apply(rank, True, x, *W)
+    dx, = torch.autograd.grad(y, [x], dy)
+    tol = 2 ** -21 + 2 ** -24 * C ** 0.5
+    rel = lambda a, b: float((a.double() - b).norm() / b.norm())
+    x64, dy64 = x.detach().double(), dy.double()
+    assert rel(y.detach(), sum(x_k @ w.detach().double().t() for x_k, w in zip(x64.split(C, 1), W))) <= tol
+    assert rel(dx, dy64 @ torch.cat([w.detach().double() for w in W], dim=1)) <= tol
+    for k in range(G):
+        # and one linear by itself
+        alone = diff._RowLinears.apply(rank, True, x.detach()[:, k * C:(k + 1) * C].contiguous(), W[k].detach())
+        ref = diff.tensor_linear(rank, W[k].detach(), _by_rank(x.detach()[:, k * C:(k + 1) * C], rank), sequential=True)
+        assert rel(alone, diff._component_rows(ref).double() if rank else ref.double()) <= 2 * tol
+    for k in range(1, G):                                    # the larger ones without a weight
+        few = [torch.zeros_like(w) if j < k else w.detach() for j, w in enumerate(W)]
+        assert rel(diff._RowLinears.apply(rank, True, x.detach(), *few),
+                   sum(x_j @ w.double().t() for x_j, w in zip(x64.split(C, 1), few))) <= tol, k
+
+
+@pytest.mark.parametrize("rank, C, O, N", [(1, 64, 256, 300), (1, 256, 64, 10922), (2, 256, 64, 3640), (2, 256, 16, 8000)])
+def test_component_rows_below_the_line_stay_in_fp32(pkg, rank, C, O, N):
+    """Linears on component rows keep fp32 operands below 32 768 rows and for fewer than 64 outputs, like the linears of
+    tensors: an entry 2^-30 as large as its row's largest, whose weight is zero, keeps its 24 bits (pieces of fp16 would leave it 9)."""
+    diff = importlib.import_module("learned-dynamics_amd.differentiable")
+    g = torch.Generator().manual_seed(C)
+    R = N * 3 ** rank
+    x, W = 2.0 ** -30 * torch.randn(R, C, generator=g), torch.randn(O, C, generator=g)
+    x[:, 0], W[:, 0] = 1.0, 0.0
+    y = diff._RowLinears.apply(rank, True, x.cuda(), W.cuda()).double().cpu()
+    want = x.double() @ W.double().t()
+    assert float((y - want).norm() / want.norm()) <= 2 ** -24 * (2 + C ** 0.5)
+
+
 @pytest.mark.parametrize("N,E,C", [(5, 3, 64), (37, 500, 192)])
 def test_message_gradients_by_product_and_by_component(pkg, ops, N, E, C):
     """ops.bee_message_bwd, operands and products one by one and by channel, and ops.bee_message_grad, component-major and side
@@ -1295,11 +1346,10 @@ def test_recorded_backward_without_any_gradient(pkg, what):
     rows = lambda: [rnd(N, C), rnd(N, 3, C), rnd(N, 9, C)]
     if what == "node products":
         leaves = rows() + rows()
-        out = diff._NodeProducts.apply(*leaves)[:3]
+        out = diff._NodeProducts.apply(*leaves)
     else:
         leaves = (rows() if what == "rows" else [rnd(N, C, *[3] * k) for k in range(3)]) + [rnd(E, C), rnd(E, 3)]
         out = diff._MessageProducts.apply(*leaves, graph.by_dst, graph.by_src, None, what == "by product")
-        out = out[:3] if what == "rows" else out
 
     class Drop(torch.autograd.Function):
         @staticmethod
