@@ -475,6 +475,11 @@ int mg_tensor_linear_wgrad_f16x2(const float* dy, const float* x, const float* d
 int mg_tensor_linear_wgrad_f16x2_rows(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,
                                       const float* x_bound, long n_x_bound, long rows, long bias_rows, int dim_in, int dim_out,
                                       void* workspace, float* dW, float* db /* (dim_out) or NULL */, mg_stream_t stream);
+/* the same for x = [x_0 | x_1 | ..] of `groups` operands of dim_in / groups columns (a multiple of 4), each with a scale of its own;
+ * x_rowmax (rows, groups): the row maxima of |x_p| or bounds of them */
+int mg_tensor_linear_wgrad_f16x2_groups(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,
+                                        const float* x_rowmax, int groups, long rows, int dim_in, int dim_out, void* workspace,
+                                        float* dW, mg_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Ant16 (managan/codegen_tensor_products.py:19-34; ant16_o0_cuda / ant16_o1_cuda / ant16_o2_cuda /

@@ -318,10 +318,21 @@ __global__ void __launch_bounds__(256) absmax_parts_scalar_kernel(const BoundArr
     __syncthreads();
     if (threadIdx.x == 0) parts[block] = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
 }
+// parts[g per + b] = max |x[.., g]| over the b-th share of the rows of x (rows, groups); a block (b, g)
+__global__ void __launch_bounds__(256) absmax_columns_kernel(const float* __restrict__ x, long rows, int groups, float* __restrict__ parts) {
+    float m = 0.f;
+    for (long r = (long)blockIdx.x * 256 + threadIdx.x; r < rows; r += 256L * gridDim.x) m = fmaxf(m, fabsf(x[r * groups + blockIdx.y]));
+    for (int d = 1; d < 64; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
+    __shared__ float wave_max[4];
+    if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) parts[blockIdx.y * gridDim.x + blockIdx.x] = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
+}
 
+// group_cols: columns of x that share a scale (I: all of them)
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) wgrad_f16x2_kernel(const float* __restrict__ dy, const float* __restrict__ x,
                                                           const float* __restrict__ dy_parts, int n_dy_parts,
-                                                          const float* __restrict__ x_parts, int n_x_parts,
+                                                          const float* __restrict__ x_parts, int n_x_parts, int group_cols,
                                                           long R, int I, int O, long rows_per_block,
                                                           float* __restrict__ part, float* __restrict__ colsum_part,
                                                           long bias_rows) {
@@ -333,7 +344,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     const long r_lo = (long)blockIdx.z * rows_per_block;
     const long r_hi = r_lo + rows_per_block < R ? r_lo + rows_per_block : R;
 
-    float scale = 0.f, unscale = 0.f;                      // (set by set_scales below)
+    float scale = 0.f, unscale[2] = {0.f, 0.f};            // (set by set_scales below; of this lane's two columns of dW)
     // staging role of this thread: operand (wave-uniform), 8 rows from row 8 * octet, columns 4 cq .. 4 cq + 3.
     // A stage is the 32 rows from `first`; the last stage of a slice starts at r_hi - 32, inside the matrix
     // (rows >= 32), and the rows it shares with the stage before, or with the slice before, are scaled by zero, as
@@ -401,18 +412,26 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int j = 4 * n4 + threadIdx.x; j < n; j += 256) mx = fmaxf(mx, fabsf(p[j]));
         return mx;
     };
-    float ma = absmax_of(dy_parts, n_dy_parts), mb = absmax_of(x_parts, n_x_parts);
-    for (int d = 1; d < 64; d <<= 1) { ma = fmaxf(ma, __shfl_xor(ma, d)); mb = fmaxf(mb, __shfl_xor(mb, d)); }
+    float ma = absmax_of(dy_parts, n_dy_parts);
     float* wave_max = reinterpret_cast<float*>(lds);
-    if (lane == 0) { wave_max[wave] = ma; wave_max[4 + wave] = mb; }
-    __syncthreads();
-    ma = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
-    mb = fmaxf(fmaxf(wave_max[4], wave_max[5]), fmaxf(wave_max[6], wave_max[7]));
-    __syncthreads();
-    float inv_a, inv_b;
-    const float scale_a = pow2_scale(ma, &inv_a), scale_b = pow2_scale(mb, &inv_b);
-    scale = col_ok ? (stage_x ? scale_b : scale_a) : 0.f;
-    unscale = inv_a * inv_b;
+    // a scale for every group of group_cols columns of x that the tile has a part of (n_x_parts maxima each)
+    const int last_col = i_tile + kFTile < I ? i_tile + kFTile - 1 : I - 1, my_col = i_tile + 4 * cq, out_col = i_tile + 4 * m + 2 * (wave & 1);
+    for (int p = i_tile / group_cols; p <= last_col / group_cols; p++) {
+        float mb = absmax_of(x_parts + (long)p * n_x_parts, n_x_parts);
+        for (int d = 1; d < 64; d <<= 1) { ma = fmaxf(ma, __shfl_xor(ma, d)); mb = fmaxf(mb, __shfl_xor(mb, d)); }
+        if (lane == 0) { wave_max[wave] = ma; wave_max[4 + wave] = mb; }
+        __syncthreads();
+        ma = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
+        mb = fmaxf(fmaxf(wave_max[4], wave_max[5]), fmaxf(wave_max[6], wave_max[7]));
+        __syncthreads();
+        float inv_a, inv_b;
+        const float scale_a = pow2_scale(ma, &inv_a), scale_b = pow2_scale(mb, &inv_b);
+        if (!stage_x) scale = col_ok ? scale_a : 0.f;
+        else if (col_ok && my_col / group_cols == p) scale = scale_b;
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+            if ((out_col + q) / group_cols == p) unscale[q] = inv_a * inv_b;
+    }
     };
 
     floatx16 acc[2][2];
@@ -518,7 +537,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
             for (int k = 0; k < 16; k++) {
                 const int o = o_tile + 4 * (8 * (k / 4) + 4 * g + (k % 4)) + 2 * (wave >> 1) + p;
-                if (o < O && i < I) plane[(long)o * I + i] = total[p][q][k] * unscale;
+                if (o < O && i < I) plane[(long)o * I + i] = total[p][q][k] * unscale[q];
             }
         }
 }
@@ -606,9 +625,10 @@ int mg_tensor_linear_wgrad_f16x2_supported(long rows, int dim_in, int dim_out) {
     return rows >= 4096 && dim_in >= 4 && dim_out >= 4 && dim_in % 4 == 0 && dim_out % 4 == 0;
 }
 
-int mg_tensor_linear_wgrad_f16x2_rows(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,
-                                      const float* x_bound, long n_x_bound, long rows, long bias_rows, int dim_in, int dim_out,
-                                      void* workspace, float* dW, float* db, mg_stream_t stream) {
+// groups > 1: x_bound holds (rows, groups) maxima, one of each dim_in / groups columns
+static int wgrad_f16x2(const float* dy, const float* x, const float* dy_bound, long n_dy_bound, const float* x_bound, long n_x_bound,
+                       int groups, long rows, long bias_rows, int dim_in, int dim_out, void* workspace, float* dW, float* db,
+                       mg_stream_t stream) {
     MG_REQUIRE(mg_tensor_linear_wgrad_f16x2_supported(rows, dim_in, dim_out),
                "mg_tensor_linear_wgrad_f16x2: needs rows >= 4096 and dims that are multiples of 4");
     MG_REQUIRE(dy && x && workspace && dW, "mg_tensor_linear_wgrad_f16x2: null pointer");
@@ -637,20 +657,42 @@ int mg_tensor_linear_wgrad_f16x2_rows(const float* dy, const float* x, const flo
         return blocks;
     };
     const int na = bound_parts(scan[0], dy, rows * dim_out, dy_bound, n_dy_bound, maxima);
-    const int nb = bound_parts(scan[1], x, rows * dim_in, x_bound, n_x_bound, maxima + kFParts);
+    int nb;
+    if (groups > 1) {
+        const long per = kFParts / groups;
+        nb = (int)(ceil_div(rows, 1024) < per ? ceil_div(rows, 1024) : per);
+        hipLaunchKernelGGL(absmax_columns_kernel, dim3((unsigned)nb, (unsigned)groups), dim3(256), 0, st, x_bound, rows, groups, maxima + kFParts);
+    } else {
+        nb = bound_parts(scan[1], x, rows * dim_in, x_bound, n_x_bound, maxima + kFParts);
+    }
     if (scan[0].blocks + scan[1].blocks > 0)
         hipLaunchKernelGGL(absmax_parts_scalar_kernel, dim3((unsigned)(scan[0].blocks + scan[1].blocks)), dim3(256), 0, st, scan[0],
                            scan[1]);
     const float* dy_parts = (dy_bound && n_dy_bound <= kDirectBounds) ? dy_bound : maxima;
-    const float* x_parts = (x_bound && n_x_bound <= kDirectBounds) ? x_bound : maxima + kFParts;
+    const float* x_parts = (groups == 1 && x_bound && n_x_bound <= kDirectBounds) ? x_bound : maxima + kFParts;
     dim3 grid((unsigned)ceil_div(dim_out, kFTile), (unsigned)ceil_div(dim_in, kFTile), (unsigned)splits), block(256);
-    hipLaunchKernelGGL(wgrad_f16x2_kernel, grid, block, 0, st, dy, x, dy_parts, na, x_parts, nb, rows, dim_in, dim_out,
-                       rpb, part, colsum_part, bias_rows);
+    hipLaunchKernelGGL(wgrad_f16x2_kernel, grid, block, 0, st, dy, x, dy_parts, na, x_parts, nb, dim_in / groups, rows, dim_in,
+                       dim_out, rpb, part, colsum_part, bias_rows);
     const long n_sum = n + (db ? dim_out : 0);
     const unsigned nblocks = (unsigned)(ceil_div(n_sum, 256) < 1024 ? ceil_div(n_sum, 256) : 1024);
     hipLaunchKernelGGL(wgrad_reduce2_kernel, dim3(nblocks), dim3(256), 0, st, (const float*)part, n, dW,
                        (const float*)colsum_part, (long)(db ? dim_out : 0), db, (int)splits);
     return check_launch("mg_tensor_linear_wgrad_f16x2");
+}
+
+int mg_tensor_linear_wgrad_f16x2_rows(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,
+                                      const float* x_bound, long n_x_bound, long rows, long bias_rows, int dim_in, int dim_out,
+                                      void* workspace, float* dW, float* db, mg_stream_t stream) {
+    return wgrad_f16x2(dy, x, dy_bound, n_dy_bound, x_bound, n_x_bound, 1, rows, bias_rows, dim_in, dim_out, workspace, dW, db, stream);
+}
+
+int mg_tensor_linear_wgrad_f16x2_groups(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,
+                                        const float* x_rowmax, int groups, long rows, int dim_in, int dim_out, void* workspace,
+                                        float* dW, mg_stream_t stream) {
+    MG_REQUIRE(groups >= 1 && groups <= kFParts && dim_in % (4 * groups) == 0 && x_rowmax,
+               "mg_tensor_linear_wgrad_f16x2_groups: groups of a multiple of four columns, and their row maxima");
+    return wgrad_f16x2(dy, x, dy_bound, n_dy_bound, x_rowmax, rows * groups, groups, rows, rows, dim_in, dim_out, workspace, dW, nullptr,
+                       stream);
 }
 
 int mg_tensor_linear_wgrad_f16x2(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,

@@ -872,7 +872,7 @@ std::tuple<OptTensor, Tensors> row_linears_bwd(const at::Tensor& dy, const at::T
     const bool f16x2 = mg_get_linear_mode() == kModeF16x2;
     const bool split_x = f16x2 && f16x2_takes(R, O, G * C, dy) && (T == 1 || component_rows_take(R, O, C, false));
     const bool split_W = f16x2 && aligned16(x) && aligned16(dy) && (T == 1 || std::max(C, O) <= 256) &&
-                         mg_tensor_linear_wgrad_f16x2_supported(R, (int)(G * C), (int)O);
+                         mg_tensor_linear_wgrad_f16x2_supported(R, (int)C, (int)O);
     OptTensor dx, dy_max;
     if ((want_x && split_x) || (want_W && split_W)) dy_max = row_absmax(dy);
     if (want_x) {
@@ -891,8 +891,8 @@ std::tuple<OptTensor, Tensors> row_linears_bwd(const at::Tensor& dy, const at::T
         at::Tensor ws = bytes_like(x, n);
         if (split_W) {
             if (!x_max.has_value()) x_max = row_absmax(x.view({R * G, C}));
-            check(mg_tensor_linear_wgrad_f16x2(fp(dy), fp(x), fp(dy_max), R, fp(x_max), R * G, R, (int)(G * C), (int)O, ws.data_ptr(),
-                                               fp(all), nullptr, stream_of(x)));
+            check(mg_tensor_linear_wgrad_f16x2_groups(fp(dy), fp(x), fp(dy_max), R, fp(x_max), (int)G, R, (int)(G * C), (int)O,
+                                                      ws.data_ptr(), fp(all), stream_of(x)));
         } else {
             check(mg_tensor_linear_wgrad(0, fp(dy), fp(x), R, (int)(G * C), (int)O, ws.data_ptr(), fp(all), stream_of(x)));
         }

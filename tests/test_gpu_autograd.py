@@ -1300,6 +1300,28 @@ def test_linears_side_by_side_of_any_magnitude(pkg, ops, rank, C, O, N):
                    sum(x_j @ w.double().t() for x_j, w in zip(x64.split(C, 1), few))) <= tol, k
 
 
+@pytest.mark.parametrize("rank, C, O, N, groups", [(0, 256, 64, 4096, 3), (0, 60, 8, 5000, 5), (0, 256, 64, 9000, 1), (1, 256, 64, 1500, 5),
+                                                   (1, 192, 132, 3000, 5), (2, 256, 16, 3001, 5), (2, 20, 12, 500, 4), (1, 256, 64, 500, 5)])
+def test_weight_gradients_side_by_side_of_any_magnitude(pkg, ops, rank, C, O, N, groups):
+    """The gradient of each weight by itself where the operands of the linears are 1 to 1e-8 in size.  Tolerance: dy and each x_k in
+    pieces of 22 bits of their own largest, M times their rms, leave an error of 2^-22 M rms / 2 per element at most, independent from
+    element to element; sums in fp32 in runs of 256, 64 such runs at most on the way to the result, add 2^-24 (16 + 8)."""
+    diff = importlib.import_module("learned-dynamics_amd.differentiable")
+    g = torch.Generator().manual_seed(N + C)
+    sizes = (1e-3, 1.0, 1e-5, 1e-6, 1e-8)[:groups]
+    R = N * 3 ** rank
+    x = torch.cat([m * torch.randn(R, C, generator=g) for m in sizes], dim=1).cuda()
+    W = [torch.randn(O, C, generator=g).cuda().requires_grad_() for _ in sizes]
+    dy = torch.randn(R, O, generator=g).cuda()
+    y = diff._RowLinears.apply(rank, True, x, *W)
+    dW = torch.autograd.grad(y, W, dy)
+    spread = lambda t: float(t.abs().max() / t.double().pow(2).mean().sqrt())
+    for k, (d, x_k) in enumerate(zip(dW, x.split(C, 1))):
+        want = dy.double().t() @ x_k.double()
+        tol = 2 ** -23 * (spread(dy) + spread(x_k)) + 2 ** -24 * 24
+        assert float((d.double() - want).norm() / want.norm()) <= tol, k
+
+
 @pytest.mark.parametrize("rank, C, O, N", [(1, 64, 256, 300), (1, 256, 64, 10922), (2, 256, 64, 3640), (2, 256, 16, 8000)])
 def test_component_rows_below_the_line_stay_in_fp32(pkg, rank, C, O, N):
     """Linears on component rows keep fp32 operands below 32 768 rows and for fewer than 64 outputs, like the linears of
