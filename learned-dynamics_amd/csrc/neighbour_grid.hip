@@ -31,7 +31,6 @@
 //   when box/cutoff is not an integer the cells are narrower than the cutoff and
 //   pairs two cells apart are not listed.
 #include "common.hpp"
-#include <type_traits>
 #include <mutex>
 #include <type_traits>
 
@@ -1121,6 +1120,7 @@ __global__ void __launch_bounds__(256) graph_fill_kernel(Grid g, Workspace w, in
     const int cap = w.hit_cap;
     const HitT* __restrict__ hits = static_cast<const HitT*>(w.hits);
     const float* __restrict__ x = out.x;
+    if (blockIdx.x == 0) graph_statistics(w, A, tiled, n_box, stats);      // (before its own loads, which these would wait behind)
     int hit[RW];
     float3 xi[RW];
 #pragma unroll
@@ -1130,7 +1130,6 @@ __global__ void __launch_bounds__(256) graph_fill_kernel(Grid g, Workspace w, in
         hit[k] = lane < cap ? (int)hits[r * cap + lane] : 0;     // (past the row's degree: not used)
         if (x) xi[k] = load3(x + 3 * r);
     }
-    if (blockIdx.x == 0) graph_statistics(w, A, tiled, n_box, stats);
     FillRow own;                                                  // row r0 + lane
     if (tiled) {
         own = row_of_tile(w, r0, lane, nrows);
@@ -1598,10 +1597,17 @@ int mg_graph_fill(const float* x, const void* workspace, size_t workspace_bytes,
         hipLaunchKernelGGL((graph_fill_kernel<decltype(hit), decltype(rw)::value>), dim3((unsigned)ceil_div(A, 4 * decltype(rw)::value)),
                            dim3(256), 0, st, g, w, tiled, box_max_entries(g), row_ptr, edge_counts, stats, capacity, out, order);
     };
-    // Rows that fill less than half of a wave's lanes are dealt out (131 072 rows of 26 edges: a whole search 101 us so, 103 with a wave to
-    // a row, 108 with half a wave to a row; of 52 edges 160, 146, 150)
+    // Beyond 16 384 rows (us of this kernel, a wave to a row / dealt out, and of the kernel before both, whose rows were dealt out, in
+    // brackets).  Rows that fill less than half of a wave's lanes are dealt out: 4 edges a row, 20 000 rows 9.2 / 6.5, 131 072 38 / 15;
+    // 26 edges, 32 768 rows 14.9 / 14.2, 131 072 49 / 35 (39).  Longer rows take a wave each up to 32 768 (20 000 of 52 16.3 / 22.4,
+    // 32 768 22 / 24), and are dealt out beyond (65 536 of 40 32 / 28 (30), of 80 58 / 47 (49); 98 304 of 52 60 / 55 (58)), up to where
+    // the edges outgrow the 256 MB of the memory-side cache: there whole waves write fewer pieces, if a row is one piece (131 072 of
+    // 52 98 / 107 (110), of 80 195 / 186 (189); 262 144 of 40 198 / 206 (209), of 80 409 / 409).
+    // 4097 to 16 384 rows take a wave each (4200 of 16 12.3 (14.4), of 52 13.3 (21.7); 16 384 24.1 (26.5) and 26.1 (34); of 4 edges,
+    // where the sums over the rows before are all there is, 12.4 (11.0) and 24.0 (22.2)).
     const double mean = 4.18879 * cutoff * cutoff * cutoff * nodes / ((double)box_x * box_y * box_z);
-    const bool dealt = tiled && mean <= 32;
+    const bool wave_rows = mean > 32 && (A <= 32768 || (mean <= kWave && A * mean >= 6.0e6));
+    const bool dealt = tiled && !wave_rows;
     auto with_rows = [&](auto hit) {
         if (A <= 4096) launch(hit, std::integral_constant<int, 1>{});
         else if (!dealt) launch(hit, std::integral_constant<int, 8>{});

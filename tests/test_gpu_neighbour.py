@@ -398,7 +398,8 @@ def test_arrays_of_a_graph_are_little_longer_than_its_edges(pkg):
 @pytest.mark.parametrize("batch,atoms,cutoff,side,clump", [
     (3, 5501, 4.0, 38.3, 0), (1, 16385, 4.0, 55.0, 500),       # rows shorter than half a wave: edges dealt out; some longer than a hit row
     (2, 8200, 5.0, 43.7, 0), (1, 17411, 6.0, 56.2, 400),       # a wave to a row, rows in several strides; a last tile of few rows
-    (1, 4097, 5.0, 34.7, 0), (5, 819, 5.0, 20.3, 300)])        # eight rows and one row to a wave without the scan of tiles
+    (1, 4097, 5.0, 34.7, 0), (5, 819, 5.0, 20.3, 300),         # eight rows and one row to a wave without the scan of tiles
+    (3, 11101, 5.0, 50.5, 300), (1, 131072, 6.0, 131.6, 0)])   # longer rows: dealt out beyond 32 768 of them, whole waves again for 6.8 M edges
 def test_fill_pass_by_rows_and_by_edges(pkg, batch, atoms, cutoff, side, clump):
     """Every branch of the fill pass against the two-call search (scan and fill kernels of their own): row pointer, edges in both widths,
     vectors recomputed from them."""
