@@ -221,6 +221,17 @@ def _recorded_gradients(f, inputs, needed, grads):
     return tuple(next(found) if need else None for need in needed)
 
 
+def _gradients_in_pieces(f, inputs, needed, grads):
+    """_recorded_gradients if the backward pass is recorded or an incoming gradient or a saved tensor carries a forward-mode
+    tangent, which the kernels of a backward pass know nothing of: the pieces have rules of their own for it, or refuse.  Else None."""
+    if torch.is_grad_enabled():
+        return _recorded_gradients(f, inputs, needed, grads)
+    if any(has_tangent(t) for t in (*inputs, *grads)):
+        pairs = [(None, None) if g is None else _unpack(g) for g in _recorded_gradients(f, inputs, needed, grads)]
+        return tuple(p if p is None else _dual(p.detach(), t if t is None else t.detach()) for p, t in pairs)
+    return None
+
+
 class _MlpSilu(torch.autograd.Function):
     """painn.MLP on rows, values alone or values and tangents: one call into the C++ binding for each direction (three
     linear maps and two activations; three weight gradients, two or three input gradients, two activations).  The
@@ -309,8 +320,9 @@ class _MlpLeaky(torch.autograd.Function):
         need = ctx.needs_input_grad
         if g is None:
             return (None,) * len(need)
-        if torch.is_grad_enabled():
-            return _recorded_gradients(lambda x, *p: (_mlp_leaky_rows(p, x),), (x, *params), need, (g,))
+        pieces = _gradients_in_pieces(lambda x, *p: (_mlp_leaky_rows(p, x),), (x, *params), need, (g,))
+        if pieces is not None:
+            return pieces
         g = g.contiguous()
         if g.data_ptr() % 16:
             g = g.clone()
@@ -1071,12 +1083,9 @@ class _NodeProducts(torch.autograd.Function):
     @staticmethod
     def backward(ctx, *dys):
         operands, need = ctx.saved_tensors, ctx.needs_input_grad
-        if torch.is_grad_enabled():
-            with torch.enable_grad():
-                leaves = [t if t.requires_grad else t.detach().requires_grad_() for t in operands]
-                out = _as_rows(*ops.stack_products(Bee.apply(*_by_channel(*leaves))))
-                dys = [torch.zeros_like(o) if g is None else g for o, g in zip(out, dys)]
-                grads = torch.autograd.grad(out, leaves, dys, create_graph=True)
+        pieces = _gradients_in_pieces(lambda *t: _as_rows(*ops.stack_products(Bee.apply(*_by_channel(*t)))), operands, (True,) * 6, dys)
+        if pieces is not None:
+            grads = [torch.zeros_like(x) if g is None else g for g, x in zip(pieces, operands)]
         else:
             N, C = operands[0].shape
             shapes = (N, 3, C), (N, 3, 5, C), (N, 9, 5, C)
@@ -1124,8 +1133,9 @@ class _RowLinears(torch.autograd.Function):
         need = ctx.needs_input_grad
         if dy is None:
             return (None,) * len(need)
-        if torch.is_grad_enabled():
-            return (None, None) + _recorded_gradients(lambda x, *W: (_row_linears_plain(ctx.rank, x, W),), (x, *W), need[2:], (dy,))
+        pieces = _gradients_in_pieces(lambda x, *W: (_row_linears_plain(ctx.rank, x, W),), (x, *W), need[2:], (dy,))
+        if pieces is not None:
+            return (None, None) + pieces
         dy = dy.contiguous()
         dx, dW = ops.row_linears_bwd(dy, x, W, x_max, 3 ** ctx.rank, need[2], any(need[3:]))
         return (None, None, dx) + tuple(d if nd else None for d, nd in zip(dW or [None] * len(W), need[3:]))

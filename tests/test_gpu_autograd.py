@@ -1386,3 +1386,41 @@ def test_recorded_backward_without_any_gradient(pkg, what):
     for recorded in (False, True):
         grads = torch.autograd.grad(dropped, leaves, retain_graph=True, create_graph=recorded)
         assert all(float(t.abs().max()) == 0.0 for t in grads)
+
+
+@pytest.mark.parametrize("what", ["mlp", "linears of rank 0", "linears of rank 2"])
+def test_tangent_of_an_incoming_gradient(pkg, what):
+    """A gradient that carries a forward-mode tangent through the backward passes that are kernels: they are linear in it, so the
+    tangent of the result is the gradient of the tangent (the same sums in another kernel: fp16 pieces leave 2^-21 per factor, four
+    factors deep, against entries of order one)."""
+    import torch.autograd.forward_ad as fwAD
+    diff, bee = (importlib.import_module(f"learned-dynamics_amd.{m}") for m in ("differentiable", "bee_layers"))
+    torch.manual_seed(5)
+    if what == "mlp":
+        x = torch.randn(600, 64, device="cuda", requires_grad=True)
+        y = diff.mlp_leaky(bee.MLP(64).cuda().requires_grad_(False), x)
+        assert "MlpLeaky" in type(y.grad_fn.next_functions[0][0]).__name__ + type(y.grad_fn).__name__
+    else:
+        rank = int(what[-1])
+        x = torch.randn(100 * 3 ** rank, 5 * 64, device="cuda", requires_grad=True)
+        y = diff._RowLinears.apply(rank, True, x, *(torch.randn(64, 64, device="cuda") / 8 for _ in range(5)))
+    g, g_t = torch.randn_like(y), torch.randn_like(y)
+    want, want_t = (torch.autograd.grad(y, x, t, retain_graph=True)[0] for t in (g, g_t))
+    with fwAD.dual_level():
+        dx, = torch.autograd.grad(y, x, fwAD.make_dual(g, g_t))
+        dx, dx_t = fwAD.unpack_dual(dx)
+    assert not dx.requires_grad
+    for a, b in ((dx, want), (dx_t, want_t)):
+        assert float((a - b).norm() / b.norm()) <= 4 * 2 ** -21
+
+
+def test_tangent_through_the_gradient_of_node_products_is_refused(pkg):
+    """Their derivative kernels have no rule for forward mode: an error, and not a gradient without its tangent."""
+    import torch.autograd.forward_ad as fwAD
+    diff = importlib.import_module("learned-dynamics_amd.differentiable")
+    leaves = [torch.randn(9, *shape, device="cuda", requires_grad=True) for shape in 2 * [(64,), (3, 64), (9, 64)]]
+    out = diff._NodeProducts.apply(*leaves)
+    with fwAD.dual_level():
+        dual = [fwAD.make_dual(torch.ones_like(o), torch.ones_like(o)) for o in out]
+        with pytest.raises(RuntimeError, match="orward AD|forward mode"):
+            torch.autograd.grad(out, leaves, dual)
