@@ -493,17 +493,24 @@ bool aligned_all(const Tensors& t) { return std::all_of(t.begin(), t.end(), [](c
 
 // Whether the three layers of an MLP on x (rows, k) go through one kernel (k: W[0]'s columns after zero padding).
 // A workgroup reads all three weights whatever the number of rows, about 30 us of a kernel at 128 -> 512 -> 512 -> 512 and 10 us
-// at 128 -> 128: for wide layers of few rows the three launches that split the reduction of each over the chip are faster (us,
-// one kernel / three launches: 128 -> 512 29.9 / 18.9 at 337 rows, 30.6 / 26.5 at 1021, 31.2 / 33.2 at 1400, 33.7 / 61.8
-// at 4096, 69 / 98 at 16 336; 256 -> 384 23.2 / 22.9 at 1021, 25.1 / 43.2 at 4096; 64 -> 256 12.6 / 14.2 at 64 rows, 26 / 53
-// at 16 384; 128 -> 128 9.9 / 14.2 at 64).  Distance from float64 at 128 -> 512: 2.3e-7 against 2.2..2.5e-7 with split
-// reductions, 2.75e-7 against 4.1e-7 at 16 336 rows.
-constexpr int64_t kMlpWide = 256, kMlpWideRows = 1024;
+// at 128 -> 128: for wide layers of few rows the three launches that split the reduction of each over the chip are faster, as long
+// as their workgroups of 32 rows x 64 columns are one round of it (us, one kernel / three launches: 128 -> 512 29.9 / 18.9 at 337
+// rows, 29.3 / 25.2 at 1024, 29.3 / 31.9 at 1100, 33.7 / 61.8 at 4096, 69 / 98 at 16 336; 256 -> 448 27.9 / 23.6 at 1100, 27.9 / 32.2 at
+// 1280; 256 -> 384 22.2 / 21.3 at 1100, 22.3 / 31.0 at 1408; 512 -> 384 25.6 / 23.4 and 25.5 / 33.6).  From 288 to 352 columns
+// neither is ahead before 1024 rows, and one kernel is beyond (256 -> 320 19.2 / 19.0 at 1024, 19.2 / 20.3 at 1280).  Narrower
+// layers take one kernel (64 -> 256 12.6 / 14.2 at 64 rows, 26 / 53 at 16 384; 128 -> 128 9.9 / 14.2 at 64).  Distance from float64
+// at 128 -> 512: 2.3e-7 against 2.2..2.5e-7 with split reductions, 2.75e-7 against 4.1e-7 at 16 336 rows.
+constexpr int64_t kMlpWide = 256;
+bool mlp_in_three(int64_t rows, int64_t dim) {
+    if (dim >= 384) return (rows + 31) / 32 * ((dim + 63) / 64) <= 256;
+    return dim > kMlpWide && rows < 1024;
+}
 bool packs_f16x2(const at::Tensor& W) { return W.size(1) % 32 == 0 && W.size(1) >= 64 && W.size(0) >= 8; }
 
 bool mlp_takes(int64_t rows, int64_t k, const Tensors& W, const at::Tensor& x) {
     const int64_t dim = W[0].size(0);
-    if (mg_get_linear_mode() != kModeF16x2 || rows < (dim > kMlpWide ? kMlpWideRows : 1) || k < 64 || dim < 64 || !mg_mlp_f16x2_supported((int)k, (int)dim))
+    if (mg_get_linear_mode() != kModeF16x2 || rows < 1 || mlp_in_three(rows, dim) || k < 64 || dim < 64 ||
+        !mg_mlp_f16x2_supported((int)k, (int)dim))
         return false;
     for (size_t l = 0; l < 3; l++)
         if (W[l].size(0) != dim || (l > 0 && W[l].size(1) != dim)) return false;

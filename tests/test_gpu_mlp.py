@@ -314,3 +314,11 @@ def test_two_mlps_in_one_launch(ops, rows, dim_in, dim):
     padded = torch.cat([x[:, :48], torch.zeros_like(x[:, 48:])], dim=1)
     for y in ops.filter_grids((padded, unit, narrow, b), (padded, unit, narrow, b)):
         _assert_rows(y, _formula(x[:, :48].double(), narrow, b), "zero columns")
+
+
+@pytest.mark.parametrize("rows, dim_in, dim", [(1024, 64, 512), (1025, 64, 512), (1344, 256, 384), (1345, 256, 384), (1023, 64, 320), (1024, 64, 320)])
+def test_wide_mlp_on_either_side_of_the_line(ops, rows, dim_in, dim):
+    """Three launches that split their reductions up to one round of the chip, one kernel beyond: the same tolerance."""
+    W, b = _weights(dim_in, dim)
+    x = torch.randn(rows, dim_in, generator=torch.Generator().manual_seed(rows)).cuda()
+    _assert_rows(ops.linear_chain(x, W, b, ACTS, None), _formula(x.double(), W, b), (rows, dim))
