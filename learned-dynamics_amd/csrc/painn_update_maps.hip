@@ -9,7 +9,9 @@
 // stores.  Transposition to rows, a linear with component rows and a pass over (rows, 3, 3n) / this kernel, us: 128 channels 1280
 // nodes 17.2 / 14.9, 5120 31 / 18, 16 336 65 / 30, 40 000 147 / 71; 64 channels 12.0 / 12.1, 21 / 13, 39 / 19, 73 / 37; 256 channels
 // 29 / 30, 51 / 39, 143 / 85, 343 / 222.  Of fewer nodes a kernel of ten workgroups takes longer than three launches (320 nodes
-// 9 .. 16 / 12 .. 28): the caller's line is at 1280.
+// 9 .. 16 / 12 .. 28).  The caller's line is at 1280 nodes, and at 2304 for 256 channels, whose workgroups are alone on a CU.
+// The whole update, both ways: 64 channels 35.4 / 35.3 at 1280, 40.0 / 37.2 at 2048; 128 channels 54.6 / 52.0 at 1280; 224
+// channels 87.5 / 84.6 at 1280; 256 channels 85 / 92 at 1280, 102.5 / 104 at 2048, 136.2 / 136.0 at 2304, 146 / 143.5 at 3072.
 #include "common.hpp"
 #include "rows_in_lds.hpp"
 

@@ -604,8 +604,8 @@ std::tuple<at::Tensor, at::Tensor> painn_update(const at::Tensor& x_a, const at:
     at::Tensor ip = floats(x_a, {rows, n}), cat = floats(x_a, {rows, 2 * n}), lrv, cat_max;
     if (n <= 256) cat_max = floats(x_a, {rows, 1});
     const mg_stream_t st = stream_of(x_a);
-    // the rows and widths whose component linear is the split-fp16 one, from 40 workgroups on (figures at the kernel)
-    const bool maps = mg_get_linear_mode() == kModeF16x2 && rows >= 1280 && packs_f16x2(W_lrv) &&
+    // the rows and widths whose component linear is the split-fp16 one (figures at the kernel)
+    const bool maps = mg_get_linear_mode() == kModeF16x2 && rows >= (n <= 224 ? 1280 : 2304) && packs_f16x2(W_lrv) &&
                       mg_painn_update_maps_supported((int)n) && aligned16(x_v) && aligned16(x_a);
     if (maps) {
         lrv = floats(x_a, {rows, 3, n});
