@@ -191,7 +191,7 @@ def test_mlp_summed_over_segments(ops, rows, dim_in, dim):
     assert float(((out.double() - ref).norm(dim=1) / size.clamp_min(1e-30)).max()) <= 1.5e-6
     assert not bool(out[row_ptr[1:] == row_ptr[:-1]].any())
     assert torch.equal(ops.mlp_leaky_rowsum(W[0], b[0], W[1], b[1], x, *args), out)
-    # rows and a weight that the pieces cannot carry stay in their segments
+    # rows that the pieces cannot carry stay in their segments
     x[rows // 2] *= 2.0 ** 110
     x[0, 1] = INF
     odd = ops.mlp_leaky_rowsum(W[0], b[0], W[1], b[1], x, *args)
@@ -322,3 +322,119 @@ def test_wide_mlp_on_either_side_of_the_line(ops, rows, dim_in, dim):
     W, b = _weights(dim_in, dim)
     x = torch.randn(rows, dim_in, generator=torch.Generator().manual_seed(rows)).cuda()
     _assert_rows(ops.linear_chain(x, W, b, ACTS, None), _formula(x.double(), W, b), (rows, dim))
+
+
+BAD = [(0, INF), (0, NAN), (1, INF), (1, NAN), (2, INF), (2, NAN), (2, 2.0 ** 110)]
+
+
+def _with(W, layer, value):
+    """The weights with one entry that the pieces cannot carry."""
+    W = [w.clone() for w in W]
+    W[layer][5, 3] = value
+    return W
+
+
+def _assert_like(y, ref, what):
+    """Finite where the formula in float64 is (which does not overflow where float32 would: larger than it holds counts as infinite).
+    There, row by row over the columns of ordinary size, as exact as any other result; a column made of ONE hidden value times 2^110
+    has that value's error, which is in proportion to its row and not to itself: relative to the column."""
+    finite = torch.isfinite(ref.float())
+    assert torch.equal(torch.isfinite(y), finite), what
+    large = finite.all(0) & (ref.abs().amax(0) > 2.0 ** 60)
+    cols = finite.all(0) & ~large
+    if bool(cols.any()):
+        _assert_rows(y[:, cols], ref[:, cols], what)
+    if bool(large.any()):
+        assert float(((y[:, large].double() - ref[:, large]).norm(dim=0) / ref[:, large].norm(dim=0)).max()) <= 1.5e-6, what
+
+
+@pytest.mark.parametrize("layer, value", [t for t in BAD if t[0] < 2])
+@pytest.mark.parametrize("rows, dim_in, dim", [(300, 64, 64), (4161, 128, 512)])
+def test_weights_beyond_the_pieces_summed_over_segments(ops, rows, dim_in, dim, layer, value):
+    W, b = (t[:2] for t in _weights(dim_in, dim))
+    W = _with(W, layer, value)
+    x = torch.randn(rows, dim_in, generator=torch.Generator().manual_seed(rows)).cuda()
+    row_ptr, seg = (t.cuda() for t in _segments(rows, rows))
+    n_out = row_ptr.numel() - 1
+    out = ops.mlp_leaky_rowsum(W[0], b[0], W[1], b[1], x, row_ptr.int(), seg.int(), n_out)
+    ref, _ = _layers_and_sum(x.double(), W, b, seg, n_out)
+    filled = row_ptr[1:] > row_ptr[:-1]
+    assert torch.equal(torch.isfinite(out), torch.isfinite(ref)) and not bool(out[~filled].any())
+    cols = [k for k in range(dim) if k != 5]
+    if layer == 1:
+        _, size = _layers_and_sum(x.double(), [W[0], W[1][cols]], [b[0], b[1][cols]], seg, n_out)
+        assert float(((out[:, cols].double() - ref[:, cols]).norm(dim=1) / size.clamp_min(1e-30)).max()) <= 1.5e-6
+        assert not bool(torch.isfinite(out[filled][:, 5]).any())
+    else:
+        assert not bool(torch.isfinite(out[filled]).any())
+
+
+@pytest.mark.parametrize("layer, value", BAD)
+@pytest.mark.parametrize("leaky", [False, True])
+@pytest.mark.parametrize("rows, dim", [(300, 64), (1400, 512), (8300, 512)])
+def test_weights_beyond_the_pieces_under_differentiation(ops, rows, dim, leaky, layer, value):
+    """One weight of each layer that is infinite, undefined or beyond the pieces, forward and in the gradient of x (whose hidden rows
+    are those of the finite weights, so that it is the adjoint's own products that meet it)."""
+    W, b = _weights(64, dim)
+    x = torch.randn(rows, 64, generator=torch.Generator().manual_seed(1)).cuda()
+    gy = torch.randn(rows, dim, generator=torch.Generator().manual_seed(2)).cuda()
+    Wd = torch.randn(dim, 64, generator=torch.Generator().manual_seed(3)).cuda() / 8
+    act = (lambda z: torch.nn.functional.leaky_relu(z, 0.1)) if leaky else torch.nn.functional.silu
+    bad = _with(W, layer, value)
+    h = x.double()
+    for k in range(3):
+        h = h @ bad[k].double().t() + b[k].double()
+        h = act(h) if k < 2 else h
+    if leaky:
+        y, _ = ops.mlp_leaky_fwd(x, bad + [Wd], b)
+        h = h + x.double() @ Wd.double().t()
+        _, saved = ops.mlp_leaky_fwd(x, W + [Wd], b)
+        g_x, _ = ops.mlp_leaky_bwd(gy, x, bad + [Wd], saved, True, False)
+        slopes = [torch.where(saved[1 + 2 * k] > 0, 1.0, 0.1).double() for k in range(2)]
+    else:
+        y, _, _ = ops.mlp_silu_fwd(x, None, None, bad, b, True)
+        _, _, saved = ops.mlp_silu_fwd(x, None, None, W, b, True)
+        g_x, _, _ = ops.mlp_silu_bwd(gy, None, x, None, bad, saved, True, False)
+        s = [torch.sigmoid(saved[1 + 3 * k].double()) for k in range(2)]
+        slopes = [s[k] * (1 + saved[1 + 3 * k].double() * (1 - s[k])) for k in range(2)]
+    _assert_like(y, h, "y")
+    d = gy.double() @ bad[2].double() * slopes[1]
+    d = d @ bad[1].double() * slopes[0]
+    _assert_like(g_x, d @ bad[0].double() + (gy.double() @ Wd.double() if leaky else 0), "g_x")
+
+
+@pytest.mark.parametrize("rows, dim", [(300, 64), (4200, 512)])
+def test_tangents_and_gradients_of_a_row_beyond_the_pieces(ops, rows, dim):
+    """A tangent row of the dual kernel and a gradient row of the LeakyReLU adjoint: linear in them, and no other row notices."""
+    W, b = _weights(64, dim)
+    g = torch.Generator().manual_seed(4)
+    x, x_t = torch.randn(rows, 64, generator=g).cuda(), torch.randn(rows, 64, generator=g).cuda()
+    y, y_t, _ = ops.mlp_silu_fwd(x, x_t, None, W, b, True)
+    odd = x_t.clone()
+    odd[5] *= 2.0 ** 110
+    odd[rows - 2, 3] = INF
+    same = torch.ones(rows, dtype=torch.bool, device="cuda")
+    same[[5, rows - 2]] = False
+    z, z_t, _ = ops.mlp_silu_fwd(x, odd, None, W, b, True)
+    assert torch.equal(z, y) and torch.equal(z_t[same], y_t[same]) and not bool(torch.isfinite(z_t[rows - 2]).any())
+    assert float((z_t[5].double() * 2.0 ** -110 - y_t[5].double()).norm() / y_t[5].double().norm()) <= 1.5e-6
+    Wd = torch.randn(dim, 64, generator=g).cuda() / 8
+    gy = torch.randn(rows, dim, generator=g).cuda()
+    _, saved = ops.mlp_leaky_fwd(x, W + [Wd], b)
+    clean, _ = ops.mlp_leaky_bwd(gy, x, W + [Wd], saved, True, False)
+    gy[5] *= 2.0 ** 100
+    gy[rows - 2, 3] = INF
+    g_x, _ = ops.mlp_leaky_bwd(gy, x, W + [Wd], saved, True, False)
+    assert torch.equal(g_x[same], clean[same]) and not bool(torch.isfinite(g_x[rows - 2]).any())
+    assert float((g_x[5].double() * 2.0 ** -100 - clean[5].double()).norm() / clean[5].double().norm()) <= 1.5e-6
+
+
+@pytest.mark.parametrize("layer, value", BAD)
+def test_a_weight_beyond_the_pieces_in_one_of_two_mlps(ops, layer, value):
+    unit = torch.ones(1, 1).cuda()
+    W, b = _weights(64, 96)
+    x = torch.rand(500, 64, generator=torch.Generator().manual_seed(3)).cuda()
+    bad = _with(W, layer, value)
+    one, other = ops.filter_grids((x, unit, W, b), (x, unit, bad, b))
+    assert torch.equal(one, ops.filter_grid(x, unit, W, b))
+    _assert_like(other, _formula(x.double(), bad, b), (layer, value))
