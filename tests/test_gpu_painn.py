@@ -733,7 +733,7 @@ def test_block_with_both_filter_grids_in_one_launch(pkg, E_bond, n):
     assert torch.equal(got[5], want[5]) and torch.equal(got[6], want[6])
 
 
-@pytest.mark.parametrize("rows, n", [(1280, 64), (1281, 96), (1400, 256), (1311, 128), (1300, 224)])
+@pytest.mark.parametrize("rows, n", [(1280, 64), (1281, 96), (1400, 256), (1311, 128), (1300, 224), (2305, 256)])
 def test_update_with_its_maps_in_one_kernel(pkg, rows, n):
     """The update against its formula in float64, where the three maps, the products over components and the row maxima are one
     kernel (whole blocks of 32 nodes, part of one, one wave to the channels and several).  Tolerance: sums of n terms, their products and
