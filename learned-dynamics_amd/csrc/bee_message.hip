@@ -24,8 +24,8 @@
 // 45 chan floats per node less to write, the same again less to read, and one GEMM launch less.
 //
 // Node features are read in component-major layout (node, comp, chan): the 13
-// gathers of a wave are 13 unit-stride 256-byte reads.  A lane owns one channel
-// and keeps its 60 running sums in registers; rows are summed in edge order.
+// gathers of a wave are unit-stride reads of 64 channels.  A lane owns one channel
+// and keeps its running sums in registers; rows are summed in edge order.
 #include "common.hpp"
 #include "rank2_linear.hpp"
 #include <type_traits>
@@ -84,27 +84,22 @@ __global__ void __launch_bounds__(256) bee_geometry_kernel(const float* __restri
     rhat[3 * e + 2] = sz * inv;
 }
 
-__device__ __forceinline__ void cross3(const float* a, const float* b, float* o) {
-    o[0] = a[1] * b[2] - a[2] * b[1];
-    o[1] = a[2] * b[0] - a[0] * b[2];
-    o[2] = a[0] * b[1] - a[1] * b[0];
-}
-
-// max over the wave of non-negative values, valid in lane 63: six cross-lane VALU moves (shifts within
-// rows of 16 lanes, then row broadcasts), no LDS traffic
+// max over the wave of non-negative values (NaN counts as zero), valid in lane 63: six cross-lane VALU operations (shifts within
+// rows of 16 lanes, then row broadcasts), no LDS traffic.  Such floats are ordered as their bits are, and an integer maximum
+// takes the moved operand directly: as fmaxf each step was a move, a shift, a canonicalisation and the maximum.
 __device__ __forceinline__ float wave_max_nonneg_last_lane(float v) {
-    auto step = [](float x, auto ctrl, auto row_mask) {
-        const int moved = __builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value,
-                                                      decltype(row_mask)::value, 0xf, false);
-        return fmaxf(x, __int_as_float(moved));
+    auto step = [](unsigned x, auto ctrl, auto row_mask) {
+        const unsigned moved = (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, decltype(row_mask)::value, 0xf, false);
+        return x > moved ? x : moved;
     };
-    v = step(v, std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});   // row_shr:1
-    v = step(v, std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});   // row_shr:2
-    v = step(v, std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});   // row_shr:4
-    v = step(v, std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});   // row_shr:8
-    v = step(v, std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});   // row_bcast:15
-    v = step(v, std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});   // row_bcast:31
-    return v;
+    unsigned x = __float_as_uint(fmaxf(v, 0.f));
+    x = step(x, std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});   // row_shr:1
+    x = step(x, std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});   // row_shr:2
+    x = step(x, std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});   // row_shr:4
+    x = step(x, std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});   // row_shr:8
+    x = step(x, std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});   // row_bcast:15
+    x = step(x, std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});   // row_bcast:31
+    return __uint_as_float(x);
 }
 
 __device__ __forceinline__ long uniform(long v) {
@@ -128,41 +123,143 @@ __device__ __forceinline__ __bf16 gather_row(__amdgpu_buffer_rsrc_t r, unsigned 
     return __builtin_bit_cast(__bf16, __builtin_amdgcn_raw_buffer_load_b16(r, (int)lane_bytes, (int)row_bytes, 0));
 }
 
-// T: storage type of the node features and of the outputs (float, or __bf16 with fp32 arithmetic)
-// PIPE: keep one edge of operands in flight ahead of the one being consumed (pays on long rows)
+// the arguments of a message; T: storage type of the node features and of the outputs (float, or __bf16 with fp32 arithmetic)
+template <typename T>
+struct MessageArgs {
+    const int *row_ptr, *dst, *order;
+    long n_nodes;
+    const float *rhat, *enc;
+    const T *La, *Lv, *Ld;
+    int chan;
+    const float *enc_W, *enc_b;
+    T *P0, *S1, *S2;
+    float *node_max, *edge_max;
+    const float* y2_packed;
+    int dim_d;
+    float* out_d;
+    int out_d_accumulate;
+};
+
+// largest |sum| of a (node, channel): with the other channels of a chunk a row bound for the GEMMs that read S1 / S2
+__device__ __forceinline__ float largest(const float (&s1)[15], const float (&s2)[45]) {
+    float mx = 0.f;
+#pragma unroll
+    for (int k = 0; k < 15; k++) mx = fmaxf(mx, fabsf(s1[k]));
+#pragma unroll
+    for (int k = 0; k < 45; k++) mx = fmaxf(mx, fabsf(s2[k]));
+    return mx;
+}
+
+// (streaming)
+__device__ __forceinline__ void put_row(__amdgpu_buffer_rsrc_t r, unsigned lane_bytes, unsigned row_bytes, float v) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, (int)lane_bytes, (int)row_bytes, 2);
+}
+__device__ __forceinline__ void put_row(__amdgpu_buffer_rsrc_t r, unsigned lane_bytes, unsigned row_bytes, __bf16 v) {
+    __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), r, (int)lane_bytes, (int)row_bytes, 2);
+}
+
+// The running sums of one (node, channel).  phi rh is formed once per edge and multiplies l directly; the sums 022 are symmetric and
+// 111 is the antisymmetric part of 112, so 54 values and 93 multiply-adds an edge make the 60 sums and the three products (they
+// took 122 with every product formed by itself).
+struct NodeSums {
+    float v011[3], v101[3], v121[3], v211[3], d022[6], d202[9], d112[9], d222[9], d212[9];
+    static __device__ __forceinline__ constexpr int sym(int x, int y) { return x <= y ? x * (5 - x) / 2 + y : y * (5 - y) / 2 + x; }
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int x = 0; x < 3; x++) v011[x] = v101[x] = v121[x] = v211[x] = 0.f;
+#pragma unroll
+        for (int k = 0; k < 6; k++) d022[k] = 0.f;
+#pragma unroll
+        for (int k = 0; k < 9; k++) d202[k] = d112[k] = d222[k] = d212[k] = 0.f;
+    }
+    // l: the 13 operands; p0: the three scalar products 000, 110, 220 of the edge
+    __device__ __forceinline__ void add(float phi, const float (&rh)[3], const float (&l)[13], float (&p0)[3]) {
+        const float *l1 = l + 1, *l2 = l + 4;
+        float pr[3], t[3];                                                              // phi rh, L rh
+#pragma unroll
+        for (int x = 0; x < 3; x++) {
+            pr[x] = phi * rh[x];
+            t[x] = l2[3 * x] * rh[0] + l2[3 * x + 1] * rh[1] + l2[3 * x + 2] * rh[2];
+        }
+        p0[0] = phi * l[0];
+        p0[1] = l1[0] * pr[0] + l1[1] * pr[1] + l1[2] * pr[2];
+        p0[2] = t[0] * pr[0] + t[1] * pr[1] + t[2] * pr[2];
+#pragma unroll
+        for (int x = 0; x < 3; x++) {
+            const float plx = p0[0] * rh[x];
+            v011[x] += plx;
+            v101[x] += phi * l1[x];
+            v121[x] += p0[1] * rh[x];
+            v211[x] += phi * t[x];
+#pragma unroll
+            for (int y = 0; y < 3; y++) {
+                const int k = 3 * x + y, a = 3 * x + (y + 1) % 3, b = 3 * x + (y + 2) % 3;
+                if (y >= x) d022[sym(x, y)] += plx * rh[y];
+                d202[k] += phi * l2[k];
+                d112[k] += l1[x] * pr[y];
+                d222[k] += t[x] * pr[y];
+                d212[k] += l2[a] * pr[(y + 2) % 3];                                     // (L[x,:] x phi rh)[y]
+                d212[k] -= l2[b] * pr[(y + 1) % 3];
+            }
+        }
+    }
+    // s1: label order 011, 101, 121, 211, 111; s2: 022, 202, 112, 222, 212, component xy -> 3x + y
+    __device__ __forceinline__ void rows(float (&s1)[15], float (&s2)[45]) const {
+#pragma unroll
+        for (int x = 0; x < 3; x++) {
+            const int a = (x + 1) % 3, b = (x + 2) % 3;
+            s1[x * 5] = v011[x];
+            s1[x * 5 + 1] = v101[x];
+            s1[x * 5 + 2] = v121[x];
+            s1[x * 5 + 3] = v211[x];
+            s1[x * 5 + 4] = d112[3 * a + b] - d112[3 * b + a];
+#pragma unroll
+            for (int y = 0; y < 3; y++) {
+                const int k = 3 * x + y;
+                s2[k * 5] = d022[sym(x, y)];
+                s2[k * 5 + 1] = d202[k];
+                s2[k * 5 + 2] = d112[k];
+                s2[k * 5 + 3] = d222[k];
+                s2[k * 5 + 4] = d212[k];
+            }
+        }
+    }
+};
+
+// Which items a wave takes.  Workgroup ids go round-robin over the 8 XCDs and an XCD starts its workgroups in id order as slots free
+// up: XCD x takes the x-th eighth of the items and workgroup (id >> 3) of it the four items 4 (id >> 3) .. + 3, one
+// per wave.  The waves in flight on an XCD are then a window of consecutive nodes of the processing order (cell
+// order) that slides forward, and the gathers of neighbouring atoms, which ask for the same rows, come close
+// enough in time to meet in the L2.  A persistent grid whose waves stride over the items put a different
+// system's nodes into flight at every trip: 2.66 ms against 2.37 ms at 32 x 2048 atoms, 256 channels, and 5.26
+// against 4.44 ms at 65536 atoms with 90 neighbours, 128 channels.  (Giving each XCD one 64-channel chunk, so
+// that its L2 sees a quarter of each row, was measured with both grids and is slower by 5 %.)
+// WHOLE: a workgroup's four items are whole nodes, and its four waves make the same trips (barriers)
+template <bool WHOLE>
+struct ItemsOfWave {
+    long per_xcd, first, step, local;
+    __device__ __forceinline__ explicit ItemsOfWave(long items) {
+        per_xcd = WHOLE ? (((items + 7) / 8 + 3) & ~3L) : (items + 7) / 8;
+        first = (blockIdx.x & 7) * per_xcd;
+        step = (long)(gridDim.x >> 3) * (blockDim.x / kWave);
+        local = (long)(blockIdx.x >> 3) * (blockDim.x / kWave) + threadIdx.x / kWave;
+    }
+};
+
+// Operands in registers, one edge ahead where PIPE (pays on long rows): any channel count and alignment.
 // Y2F: the rank-2 output linear is applied here (float storage, chan % 64 == 0, 1, 2 or 4 chunks, dim_d <= 16):
 // y2_packed as written by pack_rank2_weight_kernel, out_d (nodes, dim_d, 9); S2 is not touched
 template <typename T, bool PIPE, bool Y2F>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4)))
-bee_message_kernel(const int* __restrict__ row_ptr, const int* __restrict__ dst, const int* __restrict__ order,
-                   long n_nodes, const float* __restrict__ rhat, const float* __restrict__ enc,
-                   const T* __restrict__ La, const T* __restrict__ Lv, const T* __restrict__ Ld, int chan,
-                   const float* __restrict__ enc_W, const float* __restrict__ enc_b, T* __restrict__ P0,
-                   T* __restrict__ S1, T* __restrict__ S2, float* __restrict__ node_max,
-                   float* __restrict__ edge_max, const float* __restrict__ y2_packed, int dim_d,
-                   float* __restrict__ out_d, int out_d_accumulate) {
-    static_assert(!Y2F || std::is_same<T, float>::value, "the fused output linear is for float storage");
+bee_message_kernel(const MessageArgs<T> g) {
     const int lane = threadIdx.x & (kWave - 1);
-    const int chunks = (chan + kWave - 1) / kWave;
-    const long items = n_nodes * chunks;
-    const long a_bytes = n_nodes * chan * (long)sizeof(T);
-    const __amdgpu_buffer_rsrc_t rs_a = node_rows(La, a_bytes), rs_v = node_rows(Lv, 3 * a_bytes), rs_d = node_rows(Ld, 9 * a_bytes);
-    // Workgroup ids go round-robin over the 8 XCDs and an XCD starts its workgroups in id order as slots free up:
-    // XCD x takes the x-th eighth of the items and workgroup (id >> 3) of it the four items 4 (id >> 3) .. + 3, one
-    // per wave.  The waves in flight on an XCD are then a window of consecutive nodes of the processing order (cell
-    // order) that slides forward, and the gathers of neighbouring atoms, which ask for the same rows, come close
-    // enough in time to meet in the L2.  A persistent grid whose waves stride over the items put a different
-    // system's nodes into flight at every trip: 2.66 ms against 2.37 ms at 32 x 2048 atoms, 256 channels, and 5.26
-    // against 4.44 ms at 65536 atoms with 90 neighbours, 128 channels.  (Giving each XCD one 64-channel chunk, so
-    // that its L2 sees a quarter of each row, was measured with both grids and is slower by 5 %.)
-    // Y2F: a workgroup's four items must be whole nodes, and its four waves must make the same trips (barriers)
-    const long per_xcd = Y2F ? (((items + 7) / 8 + 3) & ~3L) : (items + 7) / 8;
-    const int xcd = blockIdx.x & 7;
-    const long waves_per_xcd = (long)(gridDim.x >> 3) * (blockDim.x / kWave);
-    const long wave_local = (long)(blockIdx.x >> 3) * (blockDim.x / kWave) + threadIdx.x / kWave;
-
-    for (long item_local = wave_local; item_local < per_xcd; item_local += waves_per_xcd) {
-        long item = uniform(xcd * per_xcd + item_local);
+    const int chan = g.chan, chunks = (chan + kWave - 1) / kWave;
+    const long a_bytes = g.n_nodes * chan * (long)sizeof(T);
+    const __amdgpu_buffer_rsrc_t rs_a = node_rows(g.La, a_bytes), rs_v = node_rows(g.Lv, 3 * a_bytes), rs_d = node_rows(g.Ld, 9 * a_bytes);
+    const long items = g.n_nodes * chunks;
+    const ItemsOfWave<Y2F> mine(items);
+    for (long local = mine.local; local < mine.per_xcd; local += mine.step) {
+        long item = uniform(mine.first + local);
         const bool valid = item < items;                       // uniform over the wave
         if constexpr (Y2F) {
             item = valid ? item : items - 1;                   // a wave without an item still meets the barriers
@@ -174,26 +271,22 @@ bee_message_kernel(const int* __restrict__ row_ptr, const int* __restrict__ dst,
         const int c = chunk * kWave + lane;
         const bool active = c < chan;
         const int cc = active ? c : chan - 1;   // inactive lanes shadow a valid channel, stores are masked
-        const long node = order ? (long)order[k_node] : k_node;
-        const long lo = valid ? row_ptr[node] : 0, hi = valid ? row_ptr[node + 1] : 0;
+        const long node = g.order ? (long)g.order[k_node] : k_node;
+        const long lo = valid ? g.row_ptr[node] : 0, hi = valid ? g.row_ptr[node + 1] : 0, last = hi - 1;
 
         float w[8];
 #pragma unroll
-        for (int m = 0; m < 8; m++) w[m] = enc_W[cc * 8 + m];
-        const float bias = enc_b[cc];
-
-        float s1[15], s2[45];
-#pragma unroll
-        for (int k = 0; k < 15; k++) s1[k] = 0.f;
-#pragma unroll
-        for (int k = 0; k < 45; k++) s2[k] = 0.f;
+        for (int m = 0; m < 8; m++) w[m] = g.enc_W[cc * 8 + m];
+        const float bias = g.enc_b[cc];
+        NodeSums sums;
+        sums.clear();
 
         // Software pipeline: the 13 gathered rows, the encoding and the direction of edge e + 1 are
         // requested before edge e is consumed (the gathers are L2 / fabric latency, and a wave has
         // nothing else to do while it waits), and dst of edge e + 2 one step earlier still.  The
         // look-ahead indices are clamped to the row, so no load is predicated.
         struct EdgeOps {
-            T l0, l1[3], l2[9];
+            T l[13];
             float en[8], rh[3];
         };
         const unsigned lane_off = (unsigned)cc;   // rows are addressed as (uniform base) + 32-bit lane offset
@@ -201,125 +294,261 @@ bee_message_kernel(const int* __restrict__ row_ptr, const int* __restrict__ dst,
         const unsigned row_bytes = (unsigned)chan * (unsigned)sizeof(T);
         auto fetch = [&](EdgeOps& o, long e, long j) {
             const unsigned jr = (unsigned)__builtin_amdgcn_readfirstlane((int)j) * row_bytes;   // byte offset of La[j]
-            o.l0 = gather_row(rs_a, lane_bytes, jr, T{});
+            o.l[0] = gather_row(rs_a, lane_bytes, jr, T{});
 #pragma unroll
-            for (int t = 0; t < 3; t++) o.l1[t] = gather_row(rs_v, lane_bytes, 3u * jr + (unsigned)t * row_bytes, T{});
+            for (int t = 0; t < 3; t++) o.l[1 + t] = gather_row(rs_v, lane_bytes, 3u * jr + (unsigned)t * row_bytes, T{});
 #pragma unroll
-            for (int k = 0; k < 9; k++) o.l2[k] = gather_row(rs_d, lane_bytes, 9u * jr + (unsigned)k * row_bytes, T{});
+            for (int k = 0; k < 9; k++) o.l[4 + k] = gather_row(rs_d, lane_bytes, 9u * jr + (unsigned)k * row_bytes, T{});
 #pragma unroll
-            for (int m = 0; m < 8; m++) o.en[m] = enc[8 * e + m];
+            for (int m = 0; m < 8; m++) o.en[m] = g.enc[8 * e + m];
 #pragma unroll
-            for (int t = 0; t < 3; t++) o.rh[t] = rhat[3 * e + t];
+            for (int t = 0; t < 3; t++) o.rh[t] = g.rhat[3 * e + t];
         };
-        const long last = hi - 1;
-        EdgeOps nxt;
-        long j_next = 0;
-        if (PIPE && lo < hi) {
-            fetch(nxt, lo, dst[lo]);
-            j_next = dst[lo + 1 < hi ? lo + 1 : last];
-        }
-        for (long e = lo; e < hi; e++) {
-            EdgeOps cur;
-            if constexpr (PIPE) {
-                cur = nxt;
-                const long e1 = e + 1 < hi ? e + 1 : last;
-                fetch(nxt, e1, j_next);
-                j_next = dst[e + 2 < hi ? e + 2 : last];
-            } else {
-                fetch(cur, e, dst[e]);
-            }
-            float en[8], rh[3];
+        auto consume = [&](const EdgeOps& o, long e) {
+            float l[13], p0[3], phi = bias;
 #pragma unroll
-            for (int m = 0; m < 8; m++) en[m] = cur.en[m];
+            for (int k = 0; k < 13; k++) l[k] = (float)o.l[k];
 #pragma unroll
-            for (int t = 0; t < 3; t++) rh[t] = cur.rh[t];
-            const float l0 = (float)cur.l0;
-            float l1[3], l2[9];
-#pragma unroll
-            for (int t = 0; t < 3; t++) l1[t] = (float)cur.l1[t];
-#pragma unroll
-            for (int k = 0; k < 9; k++) l2[k] = (float)cur.l2[k];
-            float phi = bias;
-#pragma unroll
-            for (int m = 0; m < 8; m++) phi += w[m] * en[m];
-
-            // geometric pieces
-            float t_[3];   // L rh
-#pragma unroll
-            for (int x = 0; x < 3; x++) t_[x] = l2[3 * x] * rh[0] + l2[3 * x + 1] * rh[1] + l2[3 * x + 2] * rh[2];
-            const float dot1 = l1[0] * rh[0] + l1[1] * rh[1] + l1[2] * rh[2];          // l1 . rh
-            const float quad = t_[0] * rh[0] + t_[1] * rh[1] + t_[2] * rh[2];           // rh^T L rh
-            float cr[3];
-            cross3(l1, rh, cr);
-            const float pl0 = phi * l0;
-            const float pd1 = phi * dot1;
-
+            for (int m = 0; m < 8; m++) phi += w[m] * o.en[m];
+            sums.add(phi, o.rh, l, p0);
             if (active) {
-                T* p = P0 + (e * 3) * chan;
                 // outputs are written once and not read back here: streaming stores leave the L2 to the gathered rows
-                __builtin_nontemporal_store((T)pl0, p + lane_off);                       // 000
-                __builtin_nontemporal_store((T)pd1, p + chan + lane_off);                // 110
-                __builtin_nontemporal_store((T)(phi * quad), p + 2 * chan + lane_off);   // 220
+                const __amdgpu_buffer_rsrc_t p = node_rows(g.P0 + (e * 3) * chan, 3L * row_bytes);
+#pragma unroll
+                for (int k = 0; k < 3; k++) put_row(p, lane_bytes, k * row_bytes, (T)p0[k]);
             }
-            if (edge_max) {
+            if (g.edge_max) {
                 // largest |P0| entry of this (edge, 64-channel chunk): a row bound for the per-edge GEMM
-                float mx = fmaxf(fmaxf(fabsf(pl0), fabsf(pd1)), fabsf(phi * quad));
-                mx = wave_max_nonneg_last_lane(active ? mx : 0.f);
-                if (lane == kWave - 1) edge_max[e * chunks + chunk] = mx;
+                const float mx = wave_max_nonneg_last_lane(active ? fmaxf(fmaxf(fabsf(p0[0]), fabsf(p0[1])), fabsf(p0[2])) : 0.f);
+                if (lane == kWave - 1) g.edge_max[e * chunks + chunk] = mx;
             }
-            // vector sums, label order 011, 101, 121, 211, 111
-#pragma unroll
-            for (int x = 0; x < 3; x++) {
-                s1[x * 5 + 0] += pl0 * rh[x];
-                s1[x * 5 + 1] += phi * l1[x];
-                s1[x * 5 + 2] += pd1 * rh[x];
-                s1[x * 5 + 3] += phi * t_[x];
-                s1[x * 5 + 4] += phi * cr[x];
+        };
+        EdgeOps cur;
+        if constexpr (PIPE) {
+            // two sets of operands in turn: no copies
+            EdgeOps nxt;
+            long j_next = 0;
+            if (lo < hi) {
+                fetch(cur, lo, g.dst[lo]);
+                j_next = g.dst[lo + 1 < hi ? lo + 1 : last];
             }
-            // rank-2 sums, label order 022, 202, 112, 222, 212 ; component xy -> 3x+y
-#pragma unroll
-            for (int x = 0; x < 3; x++) {
-                float rowx[3];
-                cross3(l2 + 3 * x, rh, rowx);   // L[x,:] x rh
-                const float pl1x = phi * l1[x];
-                const float ptx = phi * t_[x];
-#pragma unroll
-                for (int y = 0; y < 3; y++) {
-                    const int k = 3 * x + y;
-                    s2[k * 5 + 0] += pl0 * (rh[y] * rh[x]);
-                    s2[k * 5 + 1] += phi * l2[k];
-                    s2[k * 5 + 2] += pl1x * rh[y];
-                    s2[k * 5 + 3] += ptx * rh[y];
-                    s2[k * 5 + 4] += phi * rowx[y];
-                }
+            for (long e = lo; e < hi; e += 2) {
+                fetch(nxt, e + 1 < hi ? e + 1 : last, j_next);
+                j_next = g.dst[e + 2 < hi ? e + 2 : last];
+                consume(cur, e);
+                if (e + 1 >= hi) break;
+                fetch(cur, e + 2 < hi ? e + 2 : last, j_next);
+                j_next = g.dst[e + 3 < hi ? e + 3 : last];
+                consume(nxt, e + 1);
+            }
+        } else {
+            for (long e = lo; e < hi; e++) {
+                fetch(cur, e, g.dst[e]);
+                consume(cur, e);
             }
         }
+        float s1[15], s2[45];
+        sums.rows(s1, s2);
         if (active && valid) {
-            T* o1 = S1 + node * 15 * chan;
+            const __amdgpu_buffer_rsrc_t o1 = node_rows(g.S1 + node * 15 * chan, 15L * row_bytes);
 #pragma unroll
-            for (int k = 0; k < 15; k++) __builtin_nontemporal_store((T)s1[k], o1 + k * chan + lane_off);
+            for (int k = 0; k < 15; k++) put_row(o1, lane_bytes, k * row_bytes, (T)s1[k]);
             if constexpr (!Y2F) {
-                T* o2 = S2 + node * 45 * chan;
+                const __amdgpu_buffer_rsrc_t o2 = node_rows(g.S2 + node * 45 * chan, 45L * row_bytes);
 #pragma unroll
-                for (int k = 0; k < 45; k++) __builtin_nontemporal_store((T)s2[k], o2 + k * chan + lane_off);
+                for (int k = 0; k < 45; k++) put_row(o2, lane_bytes, k * row_bytes, (T)s2[k]);
             }
         }
-        if (node_max) {
-            // largest |sum| of this (node, 64-channel chunk): a row bound for the GEMMs that read S1 / S2
-            float mx = 0.f;
-#pragma unroll
-            for (int k = 0; k < 15; k++) mx = fmaxf(mx, fabsf(s1[k]));
-#pragma unroll
-            for (int k = 0; k < 45; k++) mx = fmaxf(mx, fabsf(s2[k]));
-            mx = wave_max_nonneg_last_lane(active ? mx : 0.f);
-            if (lane == kWave - 1 && valid) node_max[node * chunks + chunk] = mx;
+        if (g.node_max) {
+            const float mx = wave_max_nonneg_last_lane(active ? largest(s1, s2) : 0.f);
+            if (lane == kWave - 1 && valid) g.node_max[node * chunks + chunk] = mx;
         }
         if constexpr (Y2F) {
-            __shared__ __attribute__((aligned(16))) float tr_buf[4][16 * kTrPitch];
-            __shared__ float part[4][16 * 16];
-            rank2_linear_of_node_sums(s2, tr_buf, part, chunk, chunks, valid, y2_packed, dim_d,
-                                      out_d + node * (long)dim_d * 9, out_d_accumulate != 0);
+            __shared__ __attribute__((aligned(16))) float lds[4 * kRank2Share];
+            rank2_linear_of_node_sums<>(s2, lds, chunk, chunks, valid, g.y2_packed, g.dim_d, g.out_d + node * (long)g.dim_d * 9,
+                                         g.out_d_accumulate != 0);
         }
+    }
+}
+
+// Rows of whole chunks of 64 channels through LDS, kDepth edges ahead of the one being consumed: 16 bytes a lane go straight there,
+// no registers wait for them.  The compiler waits for every such load before any read of LDS, so they are written out and
+// counted here: a load reads its address registers when it issues and has no destination registers, nothing depends on it
+// but the wave's own slice of LDS.
+// Against operands one edge ahead in registers and 122 multiply-adds an edge (bee_message_kernel before NodeSums): 65 536 nodes with 90
+// neighbours, 128 channels of bf16, 3.28 -> 2.72 ms; 32 x 2048 with 16, 256 channels of float with the rank-2 linear, 2.19 -> 2.04 ms;
+// 2048 nodes of it 84 -> 73 us.  Three edges ahead take 2.94 ms, 2.07 ms and 78 us, two chunks a wave (two waves a SIMD) 3.34 ms,
+// 2.18 ms and 85 us.  What bounds it: bf16 by vector issue (109 instructions an edge, 0.9 of the cycles at the 2.0 GHz that the power
+// leaves); float by what it stores and gathers (without the stores of P0 1.61 ms, with every gather a hit 1.76).
+constexpr int kDepth = 2;
+typedef int intx4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ intx4 row_words(const void* base, long bytes) {
+    const unsigned long at = reinterpret_cast<unsigned long>(base);
+    return intx4{(int)(unsigned)at, (int)((at >> 32) & 0xffff), (int)(bytes > 0xffffffffL ? 0xffffffffu : (unsigned)bytes), 0x00020000};
+}
+template <int AT>
+__device__ __forceinline__ void rows_to_lds(intx4 rsrc, unsigned lane_bytes, unsigned row_bytes, unsigned lds_at) {
+    // (five wait states: an operand in scalar registers may just have been written by a vector instruction)
+    asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :: "s"(lds_at), "v"(lane_bytes), "s"(rsrc), "s"(row_bytes), "n"(AT) : "memory", "scc");
+}
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+    static_assert(N < 64, "six bits");
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
+}
+// Waits for the loads of the k-th edge of a row, `after` edges before its end.  The queue completes in order; behind those loads
+// are the loads of the edge after it and the stores of the two edges before it, fewer at the ends of the row.  Operations that are
+// not counted here only make it wait longer.
+template <int LOADS, int STORES>
+__device__ __forceinline__ void wait_for_edge(int k, int after) {
+    static_assert(kDepth == 2, "the cases below");
+    if (after >= 1) {
+        if (k >= 2) wait_vmcnt<LOADS + 2 * STORES>();
+        else if (k == 1) wait_vmcnt<LOADS + STORES>();
+        else wait_vmcnt<LOADS>();
+    } else if (k >= 2) {
+        wait_vmcnt<2 * STORES>();
+    } else {
+        wait_vmcnt<0>();
+    }
+}
+// a value that is uniform over the wave and never written while the kernel runs: a scalar load also beside the asm above
+template <typename V>
+__device__ __forceinline__ V scalar_at(const V* p) {
+    return *(const __attribute__((address_space(4))) V*)(unsigned long)p;
+}
+
+// EMAX: the edges' maxima are asked for.  Y2F: as above.
+template <typename T, bool EMAX, bool Y2F>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 5, sizeof(T) == 4 ? 4 : 5)))
+bee_message_ring_kernel(const MessageArgs<T> g) {
+    static_assert(!Y2F || std::is_same<T, float>::value, "the fused output linear is for float storage");
+    constexpr int kPart = kWave * (int)sizeof(T);                                  // bytes of a row that a wave takes
+    constexpr int kRowLanes = kPart / 16, kRowsPerLoad = kWave / kRowLanes;
+    static_assert(kRowsPerLoad == 4 || kRowsPerLoad == 8, "two loads and one row, or one and one, make nine rows");
+    constexpr int kLoads = sizeof(T) == 4 ? 5 : 4, kStores = EMAX ? 4 : 3, kSlot = 13 * kPart;
+    // each wave has a share of LDS of its own: the ring, and once it has run dry what the rank-2 linear needs
+    constexpr int kShare = Y2F && 4 * kRank2Share > kDepth * kSlot ? 4 * kRank2Share : kDepth * kSlot;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[4 * kShare];
+    unsigned char* const ring = lds + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) * kShare;
+    const unsigned ring_at = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned long)(__attribute__((address_space(3))) unsigned char*)ring);
+
+    const int lane = threadIdx.x & (kWave - 1);
+    const int chan = g.chan, chunks = chan / kWave;
+    const long items = g.n_nodes * chunks, a_bytes = g.n_nodes * chan * (long)sizeof(T);
+    const intx4 words_a = row_words(g.La, a_bytes), words_v = row_words(g.Lv, 3 * a_bytes), words_d = row_words(g.Ld, 9 * a_bytes);
+    const unsigned row_bytes = (unsigned)chan * (unsigned)sizeof(T);
+    const ItemsOfWave<Y2F> mine(items);
+    for (long local = mine.local; local < mine.per_xcd; local += mine.step) {
+        long item = uniform(mine.first + local);
+        const bool valid = item < items;                       // uniform over the wave
+        if constexpr (Y2F) {
+            item = valid ? item : items - 1;                   // a wave without an item still meets the barriers
+        } else {
+            if (!valid) break;
+        }
+        const long k_node = item / chunks;
+        const int chunk = (int)(item - k_node * chunks), c = chunk * kWave + lane;
+        const long node = g.order ? (long)scalar_at(g.order + k_node) : k_node;
+        const int lo = valid ? scalar_at(g.row_ptr + node) : 0, n = valid ? scalar_at(g.row_ptr + node + 1) - lo : 0;
+
+        // the lane's place in a load: row lane / kRowLanes of its array, 16 bytes of the chunk's part of it
+        const unsigned at = (unsigned)(lane / kRowLanes) * row_bytes + (unsigned)(chunk * kPart) + 16u * (unsigned)(lane % kRowLanes);
+        auto request = [&](int j, unsigned slot) {                                 // kLoads of them
+            const unsigned jr = (unsigned)j * row_bytes;
+            rows_to_lds<4 * kPart>(words_d, at, 9u * jr, slot);
+            if constexpr (kRowsPerLoad == 4) rows_to_lds<8 * kPart>(words_d, at, 9u * jr + 4u * row_bytes, slot);
+            if (lane < 3 * kRowLanes) {
+                rows_to_lds<kPart>(words_v, at, 3u * jr, slot);
+                if (lane < kRowLanes) {
+                    rows_to_lds<12 * kPart>(words_d, at, 9u * jr + 8u * row_bytes, slot);
+                    rows_to_lds<0>(words_a, at, jr, slot);
+                }
+            }
+        };
+        struct Uniform {
+            float en[8], rh[3];
+        };
+        const int* dst = g.dst + lo;
+        const float *enc = g.enc + 8L * lo, *rhat = g.rhat + 3L * lo;
+        auto scalars = [&](Uniform& u, int k) {
+#pragma unroll
+            for (int m = 0; m < 8; m++) u.en[m] = scalar_at(enc + 8L * k + m);
+#pragma unroll
+            for (int t = 0; t < 3; t++) u.rh[t] = scalar_at(rhat + 3L * k + t);
+        };
+
+        float w[8];
+#pragma unroll
+        for (int m = 0; m < 8; m++) w[m] = g.enc_W[c * 8 + m];
+        const float bias = g.enc_b[c];
+        NodeSums sums;
+        sums.clear();
+        const unsigned lane_bytes = (unsigned)c * (unsigned)sizeof(T);
+        T* p0_row = g.P0 + 3L * lo * chan;
+        float* emax = EMAX ? g.edge_max + (long)lo * chunks + chunk : nullptr;
+        const unsigned emax_bytes = lane == kWave - 1 ? 0u : 0x10000u;                  // (the other lanes' are out of range and dropped)
+        int slot = 0, j_next = 0;
+        auto step = [&](const Uniform& u, Uniform& u_next, int k) {
+            wait_for_edge<kLoads, kStores>(k, n - 1 - k);
+            const T* rows = reinterpret_cast<const T*>(ring + slot) + lane;
+            float l[13], p0[3], phi = bias;
+#pragma unroll
+            for (int r = 0; r < 13; r++) l[r] = (float)rows[r * kWave];
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                          // the slot has been read: it may be filled again
+            if (k + kDepth < n) request(j_next, ring_at + (unsigned)slot);
+            j_next = scalar_at(dst + (k + kDepth + 1 < n ? k + kDepth + 1 : n - 1));
+            scalars(u_next, k + 1 < n ? k + 1 : k);
+#pragma unroll
+            for (int m = 0; m < 8; m++) phi += w[m] * u.en[m];
+            sums.add(phi, u.rh, l, p0);
+            // outputs are written once and not read back here: streaming stores leave the L2 to the gathered rows
+            const __amdgpu_buffer_rsrc_t out = node_rows(p0_row, 3L * row_bytes);
+#pragma unroll
+            for (int t = 0; t < 3; t++) put_row(out, lane_bytes, t * row_bytes, (T)p0[t]);
+            if constexpr (EMAX) {
+                // largest |P0| entry of this (edge, 64-channel chunk): a row bound for the per-edge GEMM
+                const float mx = wave_max_nonneg_last_lane(fmaxf(fmaxf(fabsf(p0[0]), fabsf(p0[1])), fabsf(p0[2])));
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(mx), node_rows(emax, 4), (int)emax_bytes, 0, 0);
+                emax += chunks;
+            }
+            p0_row += 3L * chan;
+            slot = kSlot - slot;
+        };
+        if (n > 0) {
+            Uniform even, odd;
+            request(scalar_at(dst), ring_at);
+            if (n > 1) request(scalar_at(dst + 1), ring_at + kSlot);
+            j_next = scalar_at(dst + (kDepth < n ? kDepth : n - 1));
+            scalars(even, 0);
+            for (int k = 0;;) {                                                         // two sets of scalars in turn: no copies
+                step(even, odd, k);
+                if (++k == n) break;
+                step(odd, even, k);
+                if (++k == n) break;
+            }
+        }
+
+        float s1[15], s2[45];
+        sums.rows(s1, s2);
+        if (valid) {
+            const __amdgpu_buffer_rsrc_t o1 = node_rows(g.S1 + node * 15 * chan, 15L * row_bytes);
+#pragma unroll
+            for (int k = 0; k < 15; k++) put_row(o1, lane_bytes, k * row_bytes, (T)s1[k]);
+            if constexpr (!Y2F) {
+                const __amdgpu_buffer_rsrc_t o2 = node_rows(g.S2 + node * 45 * chan, 45L * row_bytes);
+#pragma unroll
+                for (int k = 0; k < 45; k++) put_row(o2, lane_bytes, k * row_bytes, (T)s2[k]);
+            }
+            if (g.node_max) {
+                const float mx = wave_max_nonneg_last_lane(largest(s1, s2));
+                if (lane == kWave - 1) g.node_max[node * chunks + chunk] = mx;
+            }
+        }
+        if constexpr (Y2F)
+            rank2_linear_of_node_sums<kShare / 4>(s2, reinterpret_cast<float*>(lds), chunk, chunks, valid, g.y2_packed, g.dim_d,
+                                                  g.out_d + node * (long)g.dim_d * 9, g.out_d_accumulate != 0);
     }
 }
 
@@ -356,30 +585,34 @@ static int launch_bee_message(const char* what, const int* row_ptr, const int* d
     MG_REQUIRE(n_edges == 0 || (dst && rhat && enc && P0), "%s: null edge operand", what);
     MG_REQUIRE((long)n_nodes * 9 * chan * (long)sizeof(T) < (1L << 32),
                "%s: the rank-2 node rows must stay below 4 GiB (32-bit row offsets)", what);
-    const long items = (long)n_nodes * ceil_div(chan, kWave);
+    const MessageArgs<T> args{row_ptr, dst, node_order, (long)n_nodes, rhat, enc, La, Lv, Ld, chan, enc_W, enc_b, P0, S1, S2,
+                              node_max, edge_max, y2_packed, dim_d, out_d, out_d_accumulate};
     // one item per wave, four per workgroup, an eighth of the items per XCD (the kernel's loop then makes one trip)
-    const long blocks = 8 * ceil_div(ceil_div(items, 8), 4);
-    MG_REQUIRE(blocks < (1L << 31), "%s: too many (node, channel chunk) items for one launch", what);
-    // rows of a few edges do not repay the pipeline's start-up (one extra set of loads per row), unless the system
-    // is so small that the chip is not filled and a row's chain of load latencies is all there is to the time
-    const bool pipe = n_edges >= 8L * n_nodes || items <= 16384;
-#define MG_BEE_LAUNCH(PIPE, Y2F)                                                                                      \
-    hipLaunchKernelGGL((bee_message_kernel<T, PIPE, Y2F>), dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, \
-                       row_ptr, dst, node_order, (long)n_nodes, rhat, enc, La, Lv, Ld, chan, enc_W, enc_b, P0, S1, S2, \
-                       node_max, edge_max, y2_packed, dim_d, out_d, out_d_accumulate)
+    auto launch = [&](auto kernel, long items) -> int {
+        const long blocks = 8 * ceil_div(ceil_div(items, 8), 4);
+        MG_REQUIRE(blocks < (1L << 31), "%s: too many (node, channel chunk) items for one launch", what);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, args);
+        return check_launch(what);
+    };
+    const long items = (long)n_nodes * ceil_div(chan, kWave);
+    // whole chunks, in 16-byte pieces
+    const bool ring = chan % kWave == 0 && aligned16(La) && aligned16(Lv) && aligned16(Ld);
     if constexpr (std::is_same<T, float>::value) {
         if (fused) {
             MG_REQUIRE(rank2_fusable(chan, dim_d), "%s: the fused rank-2 linear needs chan = 64, 128 or 256 and dim_d <= 16", what);
             MG_REQUIRE(aligned16(y2_packed), "%s: packed weight must be 16-byte aligned", what);
-            if (pipe) MG_BEE_LAUNCH(true, true);
-            else MG_BEE_LAUNCH(false, true);
-            return check_launch(what);
+            if (!ring) return launch(bee_message_kernel<T, true, true>, items);
+            return edge_max ? launch(bee_message_ring_kernel<T, true, true>, items) : launch(bee_message_ring_kernel<T, false, true>, items);
         }
     }
-    if (pipe) MG_BEE_LAUNCH(true, false);
-    else MG_BEE_LAUNCH(false, false);
-#undef MG_BEE_LAUNCH
-    return check_launch(what);
+    if (ring) {
+        if constexpr (std::is_same<T, float>::value)
+            if (edge_max) return launch(bee_message_ring_kernel<T, true, false>, items);
+        if (!edge_max) return launch(bee_message_ring_kernel<T, false, false>, items);
+    }
+    // rows of a few edges do not repay the pipeline's start-up (one extra set of loads per row), unless the system
+    // is so small that the chip is not filled and a row's chain of load latencies is all there is to the time
+    return n_edges >= 8L * n_nodes || items <= 16384 ? launch(bee_message_kernel<T, true, false>, items) : launch(bee_message_kernel<T, false, false>, items);
 }
 
 extern "C" {

@@ -214,8 +214,7 @@ node_rank2_linear_kernel(long n_nodes, int chan, const float* __restrict__ l0,
                                                                 const float* __restrict__ x_d,
                                                                 const float* __restrict__ L2t,
                                                                 const float* __restrict__ R2t, int dim_in2) {
-    __shared__ __attribute__((aligned(16))) float tr_buf[4][16 * kTrPitch];
-    __shared__ float part[4][16 * 16];
+    __shared__ __attribute__((aligned(16))) float rank2_lds[4 * kRank2Share];
     __shared__ float xd_buf[4][16 * 9];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int chunks = chan / kWave;
@@ -314,7 +313,7 @@ node_rank2_linear_kernel(long n_nodes, int chan, const float* __restrict__ l0,
 #pragma unroll
         for (int k = 0; k < 45; k++) s2[k] = 0.f;
     }
-    rank2_linear_of_node_sums(s2, tr_buf, part, chunk, chunks, valid, y2_packed, dim_d, out + node * (long)dim_d * 9);
+    rank2_linear_of_node_sums<>(s2, rank2_lds, chunk, chunks, valid, y2_packed, dim_d, out + node * (long)dim_d * 9);
 }
 
 template <typename T>

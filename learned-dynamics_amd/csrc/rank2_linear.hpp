@@ -15,16 +15,19 @@
 namespace mg {
 
 constexpr int kTrPitch = 68;   // floats per LDS row of a wave's transposition buffer (16-byte aligned rows)
+constexpr int kRank2Share = 16 * kTrPitch + 16 * 16;   // floats of LDS per wave: those rows and the wave's 9 x 16 results
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // Called by all four waves of the workgroup (it holds two barriers); valid = false: a wave without an item, whose s2
-// must be zeros.  out: this wave's node, (dim_d, 9); accumulate: the result is added to what out holds.
-__device__ __forceinline__ void rank2_linear_of_node_sums(const float (&s2)[45], float (&tr_buf)[4][16 * kTrPitch],
-                                                          float (&part)[4][16 * 16], int chunk, int chunks, bool valid,
+// must be zeros.  lds: kRank2Share floats for each wave, SHARE apart, 16-byte aligned.  out: this wave's node, (dim_d, 9);
+// accumulate: the result is added to what out holds.
+template <int SHARE = kRank2Share>
+__device__ __forceinline__ void rank2_linear_of_node_sums(const float (&s2)[45], float* lds, int chunk, int chunks, bool valid,
                                                           const float* __restrict__ y2_packed, int dim_d,
                                                           float* __restrict__ out, bool accumulate = false) {
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    float* tr = tr_buf[wave];
+    float* tr = lds + wave * SHARE;
+    float* results = tr + 16 * kTrPitch;
     const int ci = lane & 15, kk = lane >> 4;
     // rows 9 .. 15 of the matrix operand are rows of zeros, written once
 #pragma unroll
@@ -67,17 +70,17 @@ __device__ __forceinline__ void rank2_linear_of_node_sums(const float (&s2)[45],
     }
     // accumulator register q of lane l: comp 4 (l / 16) + q, output l % 16
 #pragma unroll
-    for (int q = 0; q < 4; q++) part[wave][(4 * kk + q) * 16 + ci] = (d0[q] + d1[q]) + (d2[q] + d3[q]);
+    for (int q = 0; q < 4; q++) results[(4 * kk + q) * 16 + ci] = (d0[q] + d1[q]) + (d2[q] + d3[q]);
     __syncthreads();
     if (chunk == 0 && valid) {                                  // the first wave of a node adds up its chunks
         for (int idx = lane; idx < dim_d * 9; idx += kWave) {
             const int j = idx / 9, i = idx - 9 * j;
             float sum = 0.f;
-            for (int wv = 0; wv < chunks; wv++) sum += part[wave + wv][i * 16 + j];
+            for (int wv = 0; wv < chunks; wv++) sum += results[wv * SHARE + i * 16 + j];
             out[idx] = accumulate ? out[idx] + sum : sum;
         }
     }
-    __syncthreads();                                            // before the workgroup's next use of part
+    __syncthreads();                                            // before the workgroup's next use of lds
 }
 
 inline bool rank2_fusable(int chan, int dim_d) {

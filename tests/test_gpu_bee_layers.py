@@ -2,6 +2,7 @@
 the oracle's restatement of archs/diffuser_atoms15.py (float64 oracle for the
 ill-conditioned radial encoding, see oracle test for its conditioning)."""
 import importlib
+import math
 
 import numpy as np
 import pytest
@@ -131,6 +132,49 @@ def test_bee_message_with_the_rank2_linear_inside(ops, chan, dim_d, N, E):
         wide.mul_(2.0)
     out2 = ops.bee_message(*args, Y2=Y2)[2]
     assert_parity_of(out2, lambda dt: (s2.to(dt) @ Y2.cpu().to(dt).t()).transpose(1, 2), "after the weight changed")
+
+
+@pytest.mark.parametrize("chan,bf16", [(64, False), (128, False), (256, False), (64, True), (192, True)])
+def test_bee_message_rows_of_every_short_length(ops, chan, bf16):
+    """Rows of 0 to 9 and of 33 edges, through LDS (16-byte aligned operands) and through registers (operands 4 bytes off): both do
+    the same arithmetic, so they differ by contractions alone: 2 ulp of the sum of magnitudes per edge, at most 33 edges."""
+    g = torch.Generator().manual_seed(chan)
+    lengths = torch.cat([torch.arange(10), torch.tensor([33, 0, 1, 2, 3]), torch.randperm(10, generator=g), torch.tensor([0, 0])])
+    N, E = len(lengths), int(lengths.sum())
+    row_ptr = torch.cat([torch.zeros(1), lengths.cumsum(0)]).int().cuda()
+    dst = torch.randint(0, N, (E,), generator=g).int().cuda()
+    dtype = torch.bfloat16 if bf16 else torch.float32
+
+    def operand(*shape):
+        flat = torch.randn(math.prod(shape) + 2, generator=g).to(dtype).cuda()
+        return flat[:-2].view(shape), flat.roll(2)[2:].view(shape)      # (the same numbers at 0 and 2 elements past an aligned address)
+
+    left = [operand(N, chan), operand(N, 3, chan), operand(N, 9, chan)]
+    encW, encb = (torch.randn(chan, 8, generator=g) * 0.3).cuda(), torch.randn(chan, generator=g).cuda()
+    enc, rhat = ops.bee_edge_geometry((torch.randn(E, 3, generator=g) * 2.5).cuda(), 6.0)
+    assert all(x.data_ptr() % 16 == 0 and y.data_ptr() % 16 != 0 and torch.equal(x, y) for x, y in left)
+    run = ops.bee_message_bf16 if bf16 else ops.bee_message
+    got, other = (run(row_ptr, dst, rhat, enc, *[x[k] for x in left], encW, encb) for k in (0, 1))
+    for y, z in zip(got, other):
+        assert torch.isfinite(y).all()
+        # bf16: a value near a rounding boundary may land on either side of it
+        tol = 2.0 ** -7 if bf16 else 33 * 2.0 ** -22
+        assert float((y.double() - z.double()).abs().max()) <= tol * float(z.double().abs().max())
+    if not bf16:
+        phi = enc.double() @ encW.double().t() + encb.double()
+        rh = rhat.double()
+        want = dict(zip(OP.BEE_ORDER, OP.bee(*[x[0].double().cpu()[dst.cpu().long()] if x[0].dim() == 2 else
+                                               x[0].double().cpu()[dst.cpu().long()].transpose(1, 2).reshape(E, chan, *([3] * r))
+                                               for r, x in enumerate(left)], phi.cpu(), (phi[..., None] * rh[:, None]).cpu(),
+                                             (phi[..., None, None] * rh[:, None, None] * rh[:, None, :, None]).cpu())))
+        src = torch.repeat_interleave(torch.arange(N), lengths)
+        P0, S1, S2 = (t.double().cpu() for t in got)
+        for k, lab in enumerate(("000", "110", "220")):
+            assert float((P0[:, k] - want[lab]).abs().max()) <= 1e-5 * float(want[lab].abs().max())
+        for S, labels in ((S1, ("011", "101", "121", "211", "111")), (S2, ("022", "202", "112", "222", "212"))):
+            for k, lab in enumerate(labels):
+                ref = torch.zeros(N, *want[lab].shape[1:], dtype=torch.float64).index_add_(0, src, want[lab]).flatten(2).transpose(1, 2)
+                assert float((S[:, :, k] - ref).abs().max()) <= 1e-5 * float(ref.abs().max()), lab
 
 
 def test_node_products_emit_node_maxima(ops):
