@@ -410,7 +410,8 @@ typedef struct mg_mlp_f16x2_grad {
 int mg_mlp_f16x2_supported(int dim_in, int dim);      /* returns 0 / 1, not a status */
 int mg_mlp_f16x2_forward(const mg_mlp_f16x2* args /* host */, mg_stream_t stream);
 int mg_mlp_f16x2_adjoint(const mg_mlp_f16x2_grad* args /* host */, mg_stream_t stream);
-/* Two forward calls that keep nothing, of one width `dim`, in one launch. */
+/* Forward calls that keep nothing, of one width `dim`, sixteen to a launch; two of them. */
+int mg_mlp_f16x2_forward_many(const mg_mlp_f16x2* const* args /* host */, int count, mg_stream_t stream);
 int mg_mlp_f16x2_forward_pair(const mg_mlp_f16x2* first /* host */, const mg_mlp_f16x2* second /* host */, mg_stream_t stream);
 /* Linear, LeakyReLU(0.1), Linear, LeakyReLU(0.1), Linear (archs/diffuser_atoms15.py:98-110) under differentiation, as the above:
  * x (rows, dim_in), hidden layers of `dim` columns, y (rows, dim_out), all of them multiples of 32 up to 512.  Kept per hidden layer: h =

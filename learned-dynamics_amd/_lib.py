@@ -139,6 +139,7 @@ _SIGNATURES = {
     "mg_mlp_f16x2_supported": [i32, i32],
     "mg_mlp_f16x2_forward": [vp, vp],
     "mg_mlp_f16x2_adjoint": [vp, vp],
+    "mg_mlp_f16x2_forward_many": [vp, i32, vp],
     "mg_mlp_f16x2_forward_pair": [vp, vp, vp],
     "mg_mlp_leaky_f16x2_supported": [i32, i32, i32],
     "mg_mlp_leaky_f16x2_forward": [vp, vp],

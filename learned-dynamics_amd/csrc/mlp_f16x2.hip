@@ -349,16 +349,18 @@ __global__ void __launch_bounds__(64 * kMaxWaves / NI, 4) mlp_f16x2_kernel(const
     mlp_rows<MI, NI, MODE, DUAL, LEAKY>(a, blockIdx.x, a.K > a.O ? a.K : a.O);
 }
 
-// Two MLPs whose layers are equally wide in one launch: the first `tiles` workgroups are the first one's
-struct MlpPair {
-    MlpArgs job[2];
-    unsigned tiles;
+// Several MLPs whose layers are equally wide in one launch: workgroups first[k] .. first[k + 1] - 1 are the k-th one's
+constexpr int kMany = 16;          // (2.9 KB of kernel arguments)
+struct MlpMany {
+    MlpArgs job[kMany];
+    unsigned first[kMany + 1];
     int widest;
 };
 template <int MI>
-__global__ void __launch_bounds__(64 * kMaxWaves, 4) mlp_pair_f16x2_kernel(const MlpPair p) {
-    const bool second = blockIdx.x >= p.tiles;
-    mlp_rows<MI, 1, kInfer, false, false>(p.job[second], blockIdx.x - (second ? p.tiles : 0), p.widest);
+__global__ void __launch_bounds__(64 * kMaxWaves, 4) mlp_many_f16x2_kernel(const MlpMany p) {
+    int k = 0;
+    while (blockIdx.x >= p.first[k + 1]) k++;                      // (the last one ends with the grid)
+    mlp_rows<MI, 1, kInfer, false, false>(p.job[k], blockIdx.x - p.first[k], p.widest);
 }
 
 // Linear, LeakyReLU(0.1), Linear, LeakyReLU(0.1), then the sum over the rows of each segment (seg ascending); the hidden rows stay in
@@ -566,17 +568,22 @@ int choose(const MlpArgs& a, bool dual, hipStream_t st) {
 }
 
 template <int MI>
-int launch_pair(MlpPair& p, hipStream_t st) {
-    p.widest = p.job[0].O;
-    for (const MlpArgs& a : p.job) p.widest = a.K > p.widest ? a.K : p.widest;
+int launch_many(MlpMany& p, int jobs, hipStream_t st) {
+    const int O = p.job[0].O;
+    p.widest = O;
+    long tiles = 0;
+    for (int k = 0; k < jobs; k++) {
+        p.widest = p.job[k].K > p.widest ? p.job[k].K : p.widest;
+        p.first[k] = (unsigned)tiles;
+        tiles += ceil_div(p.job[k].R, 32 * MI);
+        MG_REQUIRE(tiles <= 0x7fffffffL, "mg_mlp_f16x2_forward_many: grid too large");
+    }
+    for (int k = jobs; k <= kMany; k++) p.first[k] = (unsigned)tiles;
     const size_t lds = (size_t)32 * MI * p.widest * 4 + (kMaxWaves * 32 * MI + kMaxDim) * sizeof(float);
     if (lds > 65536)
-        MG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mlp_pair_f16x2_kernel<MI>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    const long first = ceil_div(p.job[0].R, 32 * MI), tiles = first + ceil_div(p.job[1].R, 32 * MI);
-    MG_REQUIRE(tiles <= 0x7fffffffL, "mg_mlp_f16x2_pair: grid too large");
-    p.tiles = (unsigned)first;
-    hipLaunchKernelGGL(mlp_pair_f16x2_kernel<MI>, dim3((unsigned)tiles), dim3(2 * p.job[0].O), lds, st, p);
-    return check_launch("mg_mlp_f16x2_pair");
+        MG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mlp_many_f16x2_kernel<MI>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(mlp_many_f16x2_kernel<MI>, dim3((unsigned)tiles), dim3(2 * O), lds, st, p);
+    return check_launch("mg_mlp_f16x2_forward_many");
 }
 
 // Two column blocks to a wave, so that two workgroups share a CU, where the width has them: by the width alone and not by the rows as
@@ -640,16 +647,20 @@ int mg_mlp_f16x2_forward(const mg_mlp_f16x2* p, mg_stream_t stream) {
     return keep ? choose<kTrain>(a, p->dual, (hipStream_t)stream) : choose<kInfer>(a, false, (hipStream_t)stream);
 }
 
-int mg_mlp_f16x2_forward_pair(const mg_mlp_f16x2* first, const mg_mlp_f16x2* second, mg_stream_t stream) {
-    MG_REQUIRE(first && second && first->dim == second->dim, "mg_mlp_f16x2_forward_pair: two MLPs of one width");
-    MlpPair p{};
-    const mg_mlp_f16x2* in[2] = {first, second};
+// kMany to a launch
+static int forward_many(const mg_mlp_f16x2* const* in, int jobs, hipStream_t st) {
+    if (jobs > kMany) {
+        if (int code = forward_many(in, kMany, st)) return code;
+        return forward_many(in + kMany, jobs - kMany, st);
+    }
+    MlpMany p{};
     long tiles = 0;
-    for (int k = 0; k < 2; k++) {
+    int used = 0;
+    for (int k = 0; k < jobs; k++) {
         const mg_mlp_f16x2& m = *in[k];
-        MlpArgs& a = p.job[k];
-        MG_REQUIRE(m.rows >= 0 && mg_mlp_f16x2_supported(m.dim_in, m.dim) && !m.dual && !m.z[0] && !m.h[0] && !m.x_rowmax,
-                   "mg_mlp_f16x2_forward_pair: inference only, dimensions multiples of 32 up to %d", kMaxDim);
+        MG_REQUIRE(m.rows >= 0 && mg_mlp_f16x2_supported(m.dim_in, m.dim) && m.dim == in[0]->dim && !m.dual && !m.z[0] && !m.h[0] && !m.x_rowmax,
+                   "mg_mlp_f16x2_forward_many: inference only, one width, dimensions multiples of 32 up to %d", kMaxDim);
+        MlpArgs& a = p.job[used];
         a.x = m.x;
         a.R = m.rows;
         a.K = m.dim_in;
@@ -657,16 +668,28 @@ int mg_mlp_f16x2_forward_pair(const mg_mlp_f16x2* first, const mg_mlp_f16x2* sec
         a.y = m.y;
         for (int l = 0; l < 3; l++) {
             a.bias[l] = m.bias[l];
-            MG_REQUIRE(m.packed_W[l] && (!m.bias[l] || aligned16(m.bias[l])), "mg_mlp_f16x2_forward_pair: null or unaligned weight or bias");
+            MG_REQUIRE(m.packed_W[l] && (!m.bias[l] || aligned16(m.bias[l])), "mg_mlp_f16x2_forward_many: null or unaligned weight or bias");
         }
         MG_REQUIRE(fill(a, m.packed_W, a.K, a.O, a.N) && (m.rows == 0 || (a.x && a.y && aligned16(a.x) && aligned16(a.y))),
-                   "mg_mlp_f16x2_forward_pair: null or unaligned pointer");
+                   "mg_mlp_f16x2_forward_many: null or unaligned pointer");
         tiles += ceil_div(m.rows, 32);
+        if (m.rows > 0) used++;
     }
     if (tiles == 0) return MG_OK;
     // (the line of one MLP)
-    if (tiles * (first->dim / 32) > 256 * kMaxWaves) return launch_pair<2>(p, (hipStream_t)stream);
-    return launch_pair<1>(p, (hipStream_t)stream);
+    if (tiles * (in[0]->dim / 32) > 256 * kMaxWaves) return launch_many<2>(p, used, st);
+    return launch_many<1>(p, used, st);
+}
+
+int mg_mlp_f16x2_forward_many(const mg_mlp_f16x2* const* args, int count, mg_stream_t stream) {
+    MG_REQUIRE(count >= 0 && (count == 0 || args), "mg_mlp_f16x2_forward_many: null pointer");
+    for (int k = 0; k < count; k++) MG_REQUIRE(args[k] && args[k]->dim == args[0]->dim, "mg_mlp_f16x2_forward_many: MLPs of one width");
+    return count ? forward_many(args, count, (hipStream_t)stream) : MG_OK;
+}
+
+int mg_mlp_f16x2_forward_pair(const mg_mlp_f16x2* first, const mg_mlp_f16x2* second, mg_stream_t stream) {
+    const mg_mlp_f16x2* in[2] = {first, second};
+    return mg_mlp_f16x2_forward_many(in, 2, stream);
 }
 
 int mg_mlp_f16x2_adjoint(const mg_mlp_f16x2_grad* p, mg_stream_t stream) {

@@ -507,11 +507,13 @@ bool mlp_in_three(int64_t rows, int64_t dim) {
 }
 bool packs_f16x2(const at::Tensor& W) { return W.size(1) % 32 == 0 && W.size(1) >= 64 && W.size(0) >= 8; }
 
+bool mlp_takes_rows(int64_t rows, int64_t k, int64_t dim) {
+    return mg_get_linear_mode() == kModeF16x2 && rows >= 1 && !mlp_in_three(rows, dim) && k >= 64 && dim >= 64 &&
+           mg_mlp_f16x2_supported((int)k, (int)dim);
+}
 bool mlp_takes(int64_t rows, int64_t k, const Tensors& W, const at::Tensor& x) {
     const int64_t dim = W[0].size(0);
-    if (mg_get_linear_mode() != kModeF16x2 || rows < 1 || mlp_in_three(rows, dim) || k < 64 || dim < 64 ||
-        !mg_mlp_f16x2_supported((int)k, (int)dim))
-        return false;
+    if (!mlp_takes_rows(rows, k, dim)) return false;
     for (size_t l = 0; l < 3; l++)
         if (W[l].size(0) != dim || (l > 0 && W[l].size(1) != dim)) return false;
     return aligned16(x);
@@ -671,25 +673,41 @@ at::Tensor filter_grid(const at::Tensor& enc, const at::Tensor& unit, const Tens
     return chain(h, {W[1], W[2]}, {b[1], b[2]}, {kActSilu, kActNone}, Bound{OptTensor(unit), l1, bmax});
 }
 
-// Two of them, in one launch where both go through the MLP kernel
-std::tuple<at::Tensor, at::Tensor> filter_grids(const at::Tensor& enc_0, const at::Tensor& unit_0, const Tensors& W_0, const Tensors& b_0,
-                                                const at::Tensor& enc_1, const at::Tensor& unit_1, const Tensors& W_1, const Tensors& b_1) {
-    auto takes = [&](const at::Tensor& enc, const Tensors& W, const Tensors& b) {
-        return enc.dim() == 2 && enc.size(1) >= W[0].size(1) && mlp_takes(enc.size(0), enc.size(1), W, enc) && aligned_all(b);
-    };
-    if (W_0[0].size(0) != W_1[0].size(0) || enc_0.device() != enc_1.device() || !takes(enc_0, W_0, b_0) || !takes(enc_1, W_1, b_1))
-        return {filter_grid(enc_0, unit_0, W_0, b_0), filter_grid(enc_1, unit_1, W_1, b_1)};
-    c10::hip::HIPGuardMasqueradingAsCUDA guard(enc_0.device());
-    for (const auto& [enc, W, b] : {std::tie(enc_0, W_0, b_0), std::tie(enc_1, W_1, b_1)}) {
-        check_input(enc, "enc");
-        TORCH_CHECK(W.size() == 3 && b.size() == 3, "filter_grids: three layers expected");
-        for (int l = 0; l < 3; l++) check_input(b[l], "bias");
+// Several of them, in one launch where their layers have one width that the MLP kernel takes for as many rows as they have together
+Tensors filter_grids(const Tensors& enc, const Tensors& unit, const std::vector<Tensors>& W, const std::vector<Tensors>& b) {
+    const size_t jobs = enc.size();
+    TORCH_CHECK(unit.size() == jobs && W.size() == jobs && b.size() == jobs, "filter_grids: as many encodings, weights and biases");
+    int64_t rows = 0;
+    bool together = jobs > 1;
+    for (size_t k = 0; k < jobs; k++) {
+        TORCH_CHECK(W[k].size() == 3 && b[k].size() == 3, "filter_grids: three layers expected");
+        if (enc[k].dim() == 2) rows += enc[k].size(0);
     }
-    at::Tensor y_0 = floats(enc_0, {enc_0.size(0), W_0[2].size(0)}), y_1 = floats(enc_1, {enc_1.size(0), W_1[2].size(0)});
+    for (size_t k = 0; k < jobs && together; k++)
+        together = enc[k].dim() == 2 && enc[k].size(0) > 0 && enc[k].size(1) >= W[k][0].size(1) && enc[k].device() == enc[0].device() &&
+                   W[k][0].size(0) == W[0][0].size(0) && mlp_takes(rows, enc[k].size(1), W[k], enc[k]) && aligned_all(b[k]);
+    Tensors y;
+    if (!together) {
+        for (size_t k = 0; k < jobs; k++) y.push_back(filter_grid(enc[k], unit[k], W[k], b[k]));
+        return y;
+    }
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(enc[0].device());
     Tensors planes;
-    const mg_mlp_f16x2 a = mlp_args(enc_0, W_0, b_0, y_0, planes), c = mlp_args(enc_1, W_1, b_1, y_1, planes);
-    check(mg_mlp_f16x2_forward_pair(&a, &c, stream_of(enc_0)));
-    return {y_0, y_1};
+    std::vector<mg_mlp_f16x2> args;
+    for (size_t k = 0; k < jobs; k++) {
+        check_input(enc[k], "enc");
+        for (int l = 0; l < 3; l++) {
+            TORCH_CHECK(W[k][l].is_cuda() && W[k][l].scalar_type() == at::kFloat && W[k][l].dim() == 2, "filter_grids: weights must be float32 CUDA matrices");
+            check_input(b[k][l], "bias");
+            TORCH_CHECK(b[k][l].numel() == W[k][l].size(0), "bias size mismatch");
+        }
+        y.push_back(floats(enc[k], {enc[k].size(0), W[k][2].size(0)}));
+        args.push_back(mlp_args(enc[k], W[k], b[k], y[k], planes));
+    }
+    std::vector<const mg_mlp_f16x2*> at;
+    for (const mg_mlp_f16x2& a : args) at.push_back(&a);
+    check(mg_mlp_f16x2_forward_many(at.data(), (int)jobs, stream_of(enc[0])));
+    return y;
 }
 
 // Message.forward with the filter interpolated from its grid, which is evaluated here: enc (rows, k) the grid's
@@ -737,23 +755,30 @@ std::tuple<at::Tensor, at::Tensor> painn_message_grid(const at::Tensor& row_ptr,
     return {out_a, out_v};
 }
 
-// Message.forward with the filter MLP on every edge and the filter stored (few edges: the kernels that fold its layers into
+// Message.forward with the filter MLP on every edge and the filter stored, unless the caller has it as `filters` (few edges: the kernels that fold its layers into
 // the edge kernel are made for tiles of 256 edges)
 std::tuple<at::Tensor, at::Tensor> painn_message_edges(const at::Tensor& row_ptr, const at::Tensor& dst, const at::Tensor& r_ij,
                                                        const at::Tensor& x_a, const at::Tensor& x_v, const Tensors& W_actv,
                                                        const Tensors& b_actv, const at::Tensor& unit, const Tensors& W_dist,
-                                                       const Tensors& b_dist, double rmax, double epsilon, bool residual) {
+                                                       const Tensors& b_dist, double rmax, double epsilon, bool residual,
+                                                       const OptTensor& filters) {
     const MessageArgs m = message_args(row_ptr, dst, r_ij, x_a, x_v);
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x_a.device());
     const at::Tensor flat_a = x_a.reshape({m.rows, m.n});
     check_chain(flat_a, W_actv, b_actv, kSiluMlp);
     const at::Tensor actv = chain(flat_a, W_actv, b_actv, kSiluMlp, Bound{});
-    TORCH_CHECK(actv.size(1) == 4 * m.n && W_dist.size() == 3 && W_dist[2].size(0) == 4 * m.n, "weights must end in 4n rows");
+    TORCH_CHECK(actv.size(1) == 4 * m.n, "weights must end in 4n rows");
     const mg_stream_t st = stream_of(x_a);
-    const int64_t n_rbf = W_dist[0].size(1), hidden = W_dist[0].size(0);
     at::Tensor filt;
-    const int64_t g = hidden / 4;
-    if (n_rbf <= 32 && hidden % 4 == 0 && g >= 1 && g <= 256 && 256 % g == 0) {
+    if (filters.has_value()) {
+        check_input(*filters, "filters");
+        TORCH_CHECK(filters->dim() == 2 && filters->size(0) == m.E && filters->size(1) == 4 * m.n, "filters must have shape (edges, 4n)");
+        filt = *filters;
+    }
+    TORCH_CHECK(filt.defined() || (W_dist.size() == 3 && W_dist[2].size(0) == 4 * m.n), "weights must end in 4n rows");
+    const int64_t n_rbf = filt.defined() ? 0 : W_dist[0].size(1), hidden = filt.defined() ? 0 : W_dist[0].size(0), g = hidden / 4;
+    if (filt.defined()) {
+    } else if (n_rbf <= 32 && hidden % 4 == 0 && g >= 1 && g <= 256 && 256 % g == 0) {
         at::Tensor h = floats(x_a, {m.E, hidden});
         check(mg_painn_radial_linear(fp(r_ij), m.E, (int)n_rbf, (float)rmax, fp(W_dist[0]), W_dist[0].stride(0),
                                      W_dist[0].stride(1), fp(b_dist[0]), (int)hidden, kActSilu, fp(h), st));
@@ -1558,6 +1583,7 @@ void register_ops(pybind11::module_& m) {
     m.def("linear_chain", &linear_chain);
     m.def("filter_grid", &filter_grid);
     m.def("filter_grids", &filter_grids);
+    m.def("mlp_takes_rows", &mlp_takes_rows);
     m.def("painn_update", &painn_update);
     m.def("painn_message_grid", &painn_message_grid);
     m.def("painn_message_edges", &painn_message_edges);

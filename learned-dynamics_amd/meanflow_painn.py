@@ -11,7 +11,7 @@ from . import differentiable as diff
 from . import ops
 from .denoiser import TimeEmbedding
 from .graph_layers import Graph
-from .painn import MLP, Block
+from .painn import MLP, Block, run_blocks
 from .tensor_products import TensLinear
 
 
@@ -58,7 +58,7 @@ class CPaiNN(nn.Module):
 
     def forward(self, pos, graph_bond, r_ij_bond, x_a, x_v, box, topology):
         x_a = diff.add(x_a, self.atom_embed(topology)[None])
-        pos, _, _, _, _, x_a, x_v, _ = self.blocks((pos, None, None, graph_bond, r_ij_bond, x_a, x_v, box))
+        pos, _, _, _, _, x_a, x_v, _ = run_blocks(self.blocks, (pos, None, None, graph_bond, r_ij_bond, x_a, x_v, box))
         return pos, x_a, x_v
 
 

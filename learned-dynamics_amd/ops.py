@@ -1020,9 +1020,14 @@ def filter_grid(enc, unit, weights, biases):
     return _ext.filter_grid(enc, unit, weights, biases)
 
 
-def filter_grids(first, second):
-    """filter_grid of two sets of arguments, in one launch where their layers have one width."""
-    return _ext.filter_grids(*first, *second)
+def filter_grids(*jobs):
+    """filter_grid of several sets of arguments, in one launch where their layers have one width."""
+    return _ext.filter_grids(*(list(part) for part in zip(*jobs))) if jobs else []
+
+
+def filter_together(rows, dim_in, dim):
+    """True where filter_grids takes MLPs of these dimensions, `rows` in all, in one launch."""
+    return bool(_ext.mlp_takes_rows(int(rows), int(dim_in), int(dim)))
 
 
 def painn_update(x_a, x_v, W_lrv, weights, biases, gn, residual):
@@ -1039,10 +1044,10 @@ def painn_message_grid(row_ptr, dst, r_ij, node_order, x_a, x_v, W_actv, b_actv,
                                    period, epsilon, bool(sliced), residual)
 
 
-def painn_message_edges(row_ptr, dst, r_ij, x_a, x_v, W_actv, b_actv, W_dist, b_dist, rmax, epsilon, residual):
-    """Message.forward with the filter MLP on every edge and the filter stored, in one host call."""
+def painn_message_edges(row_ptr, dst, r_ij, x_a, x_v, W_actv, b_actv, W_dist, b_dist, rmax, epsilon, residual, filters=None):
+    """Message.forward with the filter MLP on every edge and the filter stored (or given: filters, (edges, 4n)), in one host call."""
     return _ext.painn_message_edges(row_ptr, dst, r_ij, x_a, x_v, W_actv, b_actv, linear_in_unit_bound(x_a.device), W_dist,
-                                    b_dist, rmax, epsilon, residual)
+                                    b_dist, rmax, epsilon, residual, filters)
 
 
 def linear_f64(W, bias, x, act=ACT_NONE):

@@ -350,8 +350,9 @@ class Message(nn.Module):
         for TABLE_RECHECK changes of the weights before it is made again: one optimizer step moves the
         interpolation error by far less than the factor ten between TABLE_ATOL / TABLE_RTOL and the layer
         tolerance, and the check costs host synchronisations that a training step should not pay every time."""
-        params = list(self.mlp_dist.parameters())
-        stamp = ops.stamp(params, keep_unversioned=True)
+        params = _mlp_params(self.mlp_dist) if type(self.mlp_dist) is MLP else None
+        # (a walk over the modules is 15 us)
+        stamp = ops.stamp(self.mlp_dist.parameters() if params is None else [*params[0], *params[1]], keep_unversioned=True)
         cache = self.__dict__.setdefault("_table_cache", {})
         if cache.get("stamp") != stamp:
             training = diff.wants_grad(self.mlp_dist)
@@ -377,21 +378,26 @@ class Message(nn.Module):
     def _sliced(self, rows, n):
         return 0 < rows <= ops.PAINN_SLICED_MAX_ROWS and n % ops.PAINN_SLICE == 0 and self.use_sliced
 
-    def forward(self, graph: Graph, x_a, x_v, r_ij, residual=False, table=None):
+    def _folds(self, E, n):
+        return E >= self.FOLD_EDGES and ops.painn_filter_message_supported(n, 4 * n, E)
+
+    def forward(self, graph: Graph, x_a, x_v, r_ij, residual=False, table=None, filters=None):
         """x_a: (batch, atoms, n), x_v: (batch, atoms, n, 3), r_ij: (edges, 3).
         Returns (dx_a, dx_v), or (x_a + dx_a, x_v + dx_v) with residual=True.  table: the filter's grid of this call
-        (filter_table of the rows that _grid_rows names), if the caller has it already."""
+        (filter_table of the rows that _grid_rows names), filters: the filter of every edge where no grid is read, if the
+        caller has it already."""
         if diff.wants_grad(self, x_a, x_v, r_ij):
             da, dv = diff.painn_message(self, graph, x_a, x_v, r_ij)
             return (diff.add(x_a, da), diff.add(x_v, dv)) if residual else (da, dv)
         B, N, n = x_a.shape
         x_a, x_v, r_ij = x_a.contiguous(), x_v.contiguous(), r_ij.contiguous()
         E = r_ij.shape[0]
-        actv_mlp, dist_mlp = _plain_params(self.mlp_actv), _plain_params(self.mlp_dist) if table is None else None
-        plain = actv_mlp is not None and (dist_mlp is not None or table is not None)
+        given = table is not None or filters is not None
+        actv_mlp, dist_mlp = _plain_params(self.mlp_actv), None if given else _plain_params(self.mlp_dist)
+        plain = actv_mlp is not None and (dist_mlp is not None or given)
         flat_a, flat_v = x_a.reshape(B * N, n), x_v.reshape(B * N, n, 3)
         res_a, res_v = (flat_a, flat_v) if residual else (None, None)
-        rows = self._grid_rows(E, n) if table is None else table.shape[0]
+        rows = table.shape[0] if table is not None else 0 if filters is not None else self._grid_rows(E, n)
         if rows:
             sliced = self._sliced(rows, n)
             if not plain:
@@ -417,14 +423,14 @@ class Message(nn.Module):
             # row_ptr, are valid; the per-edge GEMMs below would also process the rows past the edge count
             raise RuntimeError("Message.forward on a capacity-sized graph needs the filter-grid path "
                                "(n a multiple of 16, a grid accepted for these weights, edge capacity >= 4 x grid rows)")
-        fold = E >= self.FOLD_EDGES and ops.painn_filter_message_supported(n, 4 * n, E)
+        fold = filters is None and self._folds(E, n)
         if plain and not fold:
-            return ops.painn_message_edges(graph.row_ptr, graph.dst32, r_ij, x_a, x_v, *actv_mlp, *dist_mlp, self.r0,
-                                           self.epsilon, residual)
+            return ops.painn_message_edges(graph.row_ptr, graph.dst32, r_ij, x_a, x_v, *actv_mlp, *(dist_mlp or ([], [])), self.r0,
+                                           self.epsilon, residual, filters)
         actv = self.mlp_actv(flat_a)
         if dist_mlp is None or not fold:
-            out_a, out_v = ops.painn_message(graph.row_ptr, graph.dst32, r_ij, self.filters(r_ij), actv, flat_v, self.epsilon,
-                                             res_a, res_v)
+            out_a, out_v = ops.painn_message(graph.row_ptr, graph.dst32, r_ij, self.filters(r_ij) if filters is None else filters,
+                                             actv, flat_v, self.epsilon, res_a, res_v)
             return out_a.reshape(B, N, n), out_v.reshape(B, N, n, 3)
         # the filter's last layer runs inside the edge kernel: the (edges, 4n) filter is never stored
         first, second = self.mlp_dist.layers[0], self.mlp_dist.layers[2]
@@ -442,6 +448,71 @@ class Message(nn.Module):
         return out_a.reshape(B, N, n), out_v.reshape(B, N, n, 3)
 
 
+# Bytes of the filters of several blocks that are evaluated ahead of the messages that read them
+FILTERS_AHEAD = 3 << 25
+
+
+def filters_of(blocks, x_a, x_v, r_ij_bond, r_ij):
+    """What the messages of `blocks` read of their filters on one pair of graphs, as the keyword arguments of their calls, a pair
+    (message_bond, message) a block, evaluated together: a filter does not depend on the features.  The two grids of one block,
+    and the filters of every edge of all of them up to FILTERS_AHEAD: 4096 rows of a grid are half the chip (128 workgroups; two
+    in a launch 50 us, one after the other 87), the filters of 6000 edges 190 workgroups and 34 us a block, those of 700 three
+    launches; five blocks of both are 145 us.  (The grids of all blocks ahead took 60 us less than block by block for seven
+    of them, and 130 us more in the kernels that then find neither a grid nor the rows beside it in the L2.)
+    Empty where a message makes its own: recorded for differentiation, without an MLP that the kernel takes or with a grid it keeps,
+    or called with hooks, which see its arguments."""
+    n = x_a.shape[2]
+    none = [({}, {})] * len(blocks)
+    messages = [m for b in blocks for m in (b._modules["message_bond"], b._modules["message"])]
+    if (any(diff.wants_grad(b, x_a, x_v, r_ij_bond, r_ij) for b in (blocks if torch.is_grad_enabled() else blocks[:1]))
+            or not all(diff.plain_call(m, Message) for m in messages)):
+        return none
+    jobs, ahead = [], 0
+    for k, m in enumerate(messages):
+        edges = (r_ij_bond, r_ij)[k % 2]
+        E = edges.shape[0]
+        params = None if m.keep_table else _plain_params(m.mlp_dist)
+        rows = m._grid_rows(E, n) if params is not None else 0
+        if rows:
+            if len(blocks) == 1:
+                jobs.append((k, "table", m, params, rows, None))
+        elif (params is not None and E > 0 and not m._folds(E, n) and m.n_rbf % 32 == 0
+              and not ops.painn_radial_linear_supported(m.n_rbf, params[0][0].shape[0])):
+            ahead += 16 * n * E
+            jobs.append((k, "filters", m, params, E, edges))
+    if len(jobs) < 2 or ahead > FILTERS_AHEAD or not ops.filter_together(sum(j[4] for j in jobs), 64, jobs[0][3][0][0].shape[0]):
+        return none
+    encodings, inputs = {}, []
+    for _, name, m, params, rows, edges in jobs:
+        if name == "table":
+            inputs.append(m._grid_inputs(params, rows))
+            continue
+        key = (id(edges), m.n_rbf, m.r0)
+        if key not in encodings:
+            encodings[key] = ops.painn_radial_encode(edges.contiguous(), m.n_rbf, m.r0)
+        inputs.append((encodings[key], ops.linear_in_unit_bound(edges.device), *params))
+    given = [{} for _ in messages]
+    for (k, name, *_), y in zip(jobs, ops.filter_grids(*inputs)):
+        given[k] = {name: y}
+    return [tuple(given[k:k + 2]) for k in range(0, len(given), 2)]
+
+
+def run_blocks(blocks, tup):
+    """blocks(tup), blocks an nn.Sequential of Block: where they keep the positions, the filters of every edge of all of them together."""
+    pos, graph, r_ij, graph_bond, r_ij_bond, x_a, x_v, box = tup
+    in_turn = list(blocks)
+    if (len(in_turn) < 2 or graph_bond is None or 16 * x_a.shape[2] * r_ij_bond.shape[0] * len(in_turn) > FILTERS_AHEAD
+            or not diff.plain_call(blocks, nn.Sequential)
+            or not all(diff.plain_call(b, Block) and not b.pos_mutable and b.r0 == in_turn[0].r0 for b in in_turn)):
+        return blocks(tup)
+    if graph is None:
+        graph, r_ij = graph_setup(in_turn[0].r0, box, pos)
+    tup = pos, graph, r_ij, graph_bond, r_ij_bond, x_a, x_v, box
+    for block, filters in zip(in_turn, filters_of(in_turn, x_a, x_v, r_ij_bond, r_ij)):
+        tup = block(tup, filters)
+    return tup
+
+
 class Block(nn.Module):
     """archs/meanflow_painn8.py:102-125.  graph_bond may be None (no bond-graph message)."""
 
@@ -455,31 +526,14 @@ class Block(nn.Module):
         if self.pos_mutable:
             self.lin_push_pos = TensLinear(1, n, 1)
 
-    def _filter_grids(self, x_a, x_v, r_ij_bond, r_ij):
-        """The two messages' filter grids as their keyword arguments, evaluated together: a grid does not depend on the
-        features, and one of 4096 rows occupies half the chip (128 workgroups; two in a launch 50 us, one after the other 87).
-        Empty where a message makes its own: recorded for differentiation, without a grid or with one it keeps, or called with
-        hooks, which see its arguments."""
-        messages, edges = (self.message_bond, self.message), (r_ij_bond.shape[0], r_ij.shape[0])
-        if (min(edges) < 4 * Message.TABLE_ROWS[0] or not all(diff.plain_call(m, Message) for m in messages)
-                or diff.wants_grad(self, x_a, x_v, r_ij_bond, r_ij)):
-            return {}, {}
-        inputs = []
-        for m, E in zip(messages, edges):
-            params = None if m.keep_table else _plain_params(m.mlp_dist)
-            rows = m._grid_rows(E, x_a.shape[2]) if params is not None else 0
-            if not rows:
-                return {}, {}
-            inputs.append(m._grid_inputs(params, rows))
-        return tuple({"table": t} for t in ops.filter_grids(*inputs))
-
-    def forward(self, tup):
+    def forward(self, tup, filters=None):
+        """filters: this block's entry of filters_of, if the caller has evaluated it."""
         pos, graph, r_ij, graph_bond, r_ij_bond, x_a, x_v, box = tup
         if graph is None:
             graph, r_ij = graph_setup(self.r0, box, pos)
         bond = pair = {}
         if graph_bond is not None:
-            bond, pair = self._filter_grids(x_a, x_v, r_ij_bond, r_ij)
+            bond, pair = filters if filters and any(filters) else filters_of([self], x_a, x_v, r_ij_bond, r_ij)[0]
             x_a, x_v = self.message_bond(graph_bond, x_a, x_v, r_ij_bond, residual=True, **bond)
         x_a, x_v = self.message(graph, x_a, x_v, r_ij, residual=True, **pair)
         x_a, x_v = self.update(x_a, x_v, residual=True)

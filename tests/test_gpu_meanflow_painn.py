@@ -53,6 +53,32 @@ def test_se3ito_forward_against_oracle(pkg, mutate_pos):
         assert not bool(v[1].any())            # (s, t) = (0, 1) with positions left in place: identically zero
 
 
+@pytest.mark.parametrize("n, N, B", [(64, 150, 1), (128, 130, 2), (128, 400, 8)])
+def test_filters_of_all_blocks_together(pkg, n, N, B):
+    """A stack whose blocks' filters (of every edge, of grids, of some of both) are evaluated ahead against its blocks called one by one
+    (a hook on the stack that changes nothing): rows of the same arithmetic, reduced in two orders, 2^-22 of a row each, through
+    two or three blocks."""
+    r0, box = 5.0, (40.0,) * 3
+    mp, model, _ = _model(n, N, (1, 3), r0, False, seed=0x947 + n)
+    x0, one_hot, bs, bd = _system(B, N, 25.0, seed=3)
+    x1 = x0 + 0.4 * torch.randn(B, N, 3, generator=torch.Generator().manual_seed(4))
+    topo = mp.Topology(one_hot.cuda(), bs.cuda(), bd.cuda())
+    st = (torch.zeros(B).cuda(), torch.full((B,), 0.4).cuda())
+    stack = model.cpainn_1
+    graph_bond = mp.get_bond_graph(B, topo, torch.device("cuda"))
+    flat = x1.cuda().reshape(-1, 3)
+    r_bond = (flat[graph_bond.dst] - flat[graph_bond.src]).contiguous()
+    x_a, x_v = torch.randn(B, N, n).cuda(), torch.randn(B, N, n, 3).cuda()
+    with torch.no_grad():
+        got = stack(x1.cuda(), graph_bond, r_bond, x_a, x_v, box, topo)
+        hook = stack.blocks.register_forward_hook(lambda *a: None)
+        want = stack(x1.cuda(), graph_bond, r_bond, x_a, x_v, box, topo)
+        hook.remove()
+        assert torch.isfinite(model(st, x0.cuda(), x1.cuda(), box, topo)).all()
+    for y, z in zip(got[1:], want[1:]):
+        assert float((y - z).norm()) <= 2e-6 * float(z.norm())
+
+
 def test_meanflow_rollout_against_oracle(pkg):
     """Three frames of ModelPredictor.predict around Meanflow.generate with pos_mutable blocks (otherwise the
     network's output at (0, 1) is zero and the frames are just accumulated noise), the normal draws shared."""

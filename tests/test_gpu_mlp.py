@@ -316,6 +316,19 @@ def test_two_mlps_in_one_launch(ops, rows, dim_in, dim):
         _assert_rows(y, _formula(x[:, :48].double(), narrow, b), "zero columns")
 
 
+@pytest.mark.parametrize("rows, dim", [((700, 1, 33, 4096), 128), ((672,) * 5 + (6100,) * 5, 512), ((64,) * 17 + (3000,), 256), ((5, 0, 9), 512)])
+def test_many_mlps_in_one_launch(ops, rows, dim):
+    """As many as sixteen and more, one set of rows under several weights, none at all: each as by itself."""
+    unit = torch.ones(1, 1).cuda()
+    x = torch.rand(max(rows), 64, generator=torch.Generator().manual_seed(dim)).cuda() * 2 - 1
+    jobs = [(x[:r], unit, *_weights(64, dim, seed=k)) for k, r in enumerate(rows)]
+    for r, y, (x_k, _, W, b) in zip(rows, ops.filter_grids(*jobs), jobs):
+        assert y.shape == (r, dim)
+        if r:
+            _assert_rows(y, _formula(x_k.double(), W, b), (r, dim))
+    assert len(ops.filter_grids()) == 0
+
+
 @pytest.mark.parametrize("rows, dim_in, dim", [(1024, 64, 512), (1025, 64, 512), (1344, 256, 384), (1345, 256, 384), (1023, 64, 320), (1024, 64, 320)])
 def test_wide_mlp_on_either_side_of_the_line(ops, rows, dim_in, dim):
     """Three launches that split their reductions up to one round of the chip, one kernel beyond: the same tolerance."""
