@@ -26,7 +26,7 @@ inline int check_launch(const char* what) {
     return MG_OK;
 }
 
-inline long ceil_div(long a, long b) { return (a + b - 1) / b; }
+__host__ __device__ inline long ceil_div(long a, long b) { return (a + b - 1) / b; }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 

@@ -47,6 +47,15 @@ __device__ __forceinline__ HalfSplit4 split(float4 v, float s) {
     return r;
 }
 
+// Two values at a time: three instructions each (the low piece by one fused multiply-add of mixed widths; v s is exact, s a power of
+// two).
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split_pair(float v0, float v1, float s0, float s1, halfx2& hi, halfx2& lo) {
+    hi = __builtin_convertvector((floatx2{v0 * s0, v1 * s1}), halfx2);
+    lo = __builtin_convertvector((floatx2{__builtin_fmaf(v0, s0, -(float)hi[0]), __builtin_fmaf(v1, s1, -(float)hi[1])}), halfx2);
+}
+
 constexpr int kCK = 32;                     // k per chunk (two MFMA steps)
 
 // Packed planes of a weight (O, I): in the order the matrix cores read them.  A block of 32 output rows x one chunk of 32

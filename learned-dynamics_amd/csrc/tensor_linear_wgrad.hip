@@ -13,6 +13,7 @@
 // Training-side helper: not on the inference hot path.
 #include "common.hpp"
 #include "f16x2.hpp"
+#include <type_traits>
 
 namespace mg {
 namespace {
@@ -259,11 +260,19 @@ __global__ void __launch_bounds__(256) wgrad_mfma_lds_kernel(const float* __rest
 // consecutive LDS rows (as the matrix lanes read 32 consecutive rows); the epilogue undoes the permutation.  Two
 // stage buffers: while one is multiplied the next stage is split into the other and the loads of the one after are
 // in flight.
+//
+// With the splitting between the matrix instructions, three instructions a value instead of five, each load sent as soon as its
+// registers are free, no bank conflicts and a slice's tiles on one XCD, against one after the other: 512 x 512 on 155 744
+// rows 375 -> 342 us, 16 368 67 -> 59, 8192 40 -> 36; 1280 x 16 on 27 000 68 -> 61; 256 x 512 on 127 456 187 -> 168.  What bounds the
+// large ones: the parts add up as energy does, not as time (without the loads 290 us, without the LDS writes too 230,
+// reads and matrix instructions alone 218, a third of those 109); small ones a stage's chain at one wave a SIMD.
 constexpr int kFTile = 128;                        // dW tile edge
 constexpr int kFRows = 32;                         // rows per stage: two matrix steps of 16
 constexpr int kFRowW = 64;                         // bytes per LDS row: 32 halves in four 16-byte pieces, piece k of
-                                                   // row R at position k ^ ((R >> 2) & 3): 16 consecutive rows
-                                                   // touch every bank once, in writes and in reads
+                                                   // row R at position k ^ swizzle(R)
+// Rows R, R + 4, R + 8, R + 12 apart for the reads (sixteen lanes at once over 64 banks), R, R + 2, R + 4, R + 6 for the writes (eight
+// lanes over 32): no conflicts counted, a third of the LDS cycles with (R >> 2) & 3
+__device__ __forceinline__ int swizzle(int row) { return (row >> 1 & 2) | ((row >> 1 ^ row >> 3) & 1); }
 constexpr int kFPlane = kFTile * kFRowW;           // bytes of one piece of one operand
 constexpr int kFBuf = 4 * kFPlane;                 // one stage: two operands x two pieces
 constexpr int kFParts = 1024;                      // partial maxima per operand
@@ -340,8 +349,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kFBuf];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m = lane & 31, g = lane >> 5;
-    const int o_tile = blockIdx.x * kFTile, i_tile = blockIdx.y * kFTile;
-    const long r_lo = (long)blockIdx.z * rows_per_block;
+    // Workgroup ids go round-robin over the 8 XCDs: XCD x takes the x-th eighth of the (slice, tile) pairs, slice by slice, so that the
+    // tiles of a slice, which read the same rows four times over, find them in one L2
+    const int tiles_o = (int)ceil_div(O, kFTile), tiles = tiles_o * (int)ceil_div(I, kFTile);
+    const long slices = ceil_div(R, rows_per_block), per_xcd = ceil_div(slices * tiles, 8);
+    const long item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if ((blockIdx.x >> 3) >= per_xcd || item >= slices * tiles) return;
+    const long slice = item / tiles;
+    const int tile = (int)(item - slice * tiles), o_tile = tile % tiles_o * kFTile, i_tile = tile / tiles_o * kFTile;
+    const long r_lo = slice * rows_per_block;
     const long r_hi = r_lo + rows_per_block < R ? r_lo + rows_per_block : R;
 
     float scale = 0.f, unscale[2] = {0.f, 0.f};            // (set by set_scales below; of this lane's two columns of dW)
@@ -356,8 +372,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     const bool col_ok = tile0 + 4 * cq < dim;
     const float* operand = stage_x ? x : dy;                                       // (uniform)
     const unsigned lane_off = (unsigned)(8 * octet * dim + (col_ok ? tile0 + 4 * cq : 0));
-    // LDS rows cq + 32 j: their swizzle term ((row >> 2) & 3) does not depend on j
-    unsigned char* st_dst = lds + (stage_x ? 2 * kFPlane : 0) + cq * kFRowW + 16 * (octet ^ ((cq >> 2) & 3));
+    // (the swizzle of LDS rows cq + 32 j does not depend on j)
+    unsigned char* st_dst = lds + (stage_x ? 2 * kFPlane : 0) + cq * kFRowW + 16 * (octet ^ swizzle(cq));
     float4 v[8];
     auto first_row = [&](long r) { return r + kFRows <= r_hi ? r : r_hi - kFRows; };
     auto fetch = [&](long r) {
@@ -366,30 +382,47 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int u = 0; u < 8; u++) v[u] = *reinterpret_cast<const float4*>(rows + u * dim + lane_off);
     };
     // column sums of dy over the slice (the bias gradient), by the workgroups of the first column of tiles
-    const bool sum_cols = colsum_part != nullptr && blockIdx.y == 0 && !stage_x;   // (uniform)
+    const bool sum_cols = colsum_part != nullptr && i_tile == 0;                   // (uniform)
     float4 colsum = make_float4(0.f, 0.f, 0.f, 0.f);
-    auto store = [&](long r, int buf_off) {
-        const int first_live = (int)(r - first_row(r)) - 8 * octet;                // rows u >= first_live count
-        halfx8 hi[4], lo[4];
-        if (sum_cols) {
-            const long last_live = bias_rows - first_row(r) - 8 * octet;           // rows u < last_live have a bias
-#pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const bool counts = u >= first_live && u < last_live && r < r_hi;  // (selected: 0 * inf would be NaN)
-                colsum.x += counts ? v[u].x : 0.f; colsum.y += counts ? v[u].y : 0.f;
-                colsum.z += counts ? v[u].z : 0.f; colsum.w += counts ? v[u].w : 0.f;
+    // One stage in eight parts: part g splits columns 2 (g % 2) and one more of rows 2 (g / 2) and one more of the stage at r, which
+    // are in v or on their way there; every second part requests the same two rows of the stage at r_next.  finish writes the pieces.
+    struct Pieces {
+        union { halfx2 pair[4]; halfx8 all; } hi[4], lo[4];
+    };
+    auto split_part = [&](int g, Pieces& out, long r, long r_next, auto sums) {
+        const int q = g / 2, first_live = (int)(r - first_row(r)) - 8 * octet;     // rows u >= first_live count
+        const float4 v0 = v[2 * q], v1 = v[2 * q + 1];
+        const bool live[2] = {2 * q >= first_live, 2 * q + 1 >= first_live};
+        const float s0 = live[0] ? scale : 0.f, s1 = live[1] ? scale : 0.f;
+        if (g % 2 == 0) {
+            split_pair(v0.x, v1.x, s0, s1, out.hi[0].pair[q], out.lo[0].pair[q]);
+            split_pair(v0.y, v1.y, s0, s1, out.hi[1].pair[q], out.lo[1].pair[q]);
+        } else {
+            split_pair(v0.z, v1.z, s0, s1, out.hi[2].pair[q], out.lo[2].pair[q]);
+            split_pair(v0.w, v1.w, s0, s1, out.hi[3].pair[q], out.lo[3].pair[q]);
+        }
+        if constexpr (decltype(sums)::value) {                                     // (selected: 0 * inf would be NaN)
+            const long last_live = r < r_hi ? bias_rows - first_row(r) - 8 * octet : 0;    // rows u < last_live have a bias
+            const bool c0 = live[0] && 2 * q < last_live, c1 = live[1] && 2 * q + 1 < last_live;
+            if (g % 2 == 0) {
+                colsum.x += c0 ? v0.x : 0.f; colsum.y += c0 ? v0.y : 0.f;
+                colsum.x += c1 ? v1.x : 0.f; colsum.y += c1 ? v1.y : 0.f;
+            } else {
+                colsum.z += c0 ? v0.z : 0.f; colsum.w += c0 ? v0.w : 0.f;
+                colsum.z += c1 ? v1.z : 0.f; colsum.w += c1 ? v1.w : 0.f;
             }
         }
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const HalfSplit4 p = split(v[u], u >= first_live ? scale : 0.f);
-#pragma unroll
-            for (int j = 0; j < 4; j++) { hi[j][u] = p.hi[j]; lo[j][u] = p.lo[j]; }
+        if (g % 2 == 1) {
+            const float* next = operand + first_row(r_next) * dim;                 // (uniform)
+            v[2 * q] = *reinterpret_cast<const float4*>(next + 2 * q * dim + lane_off);
+            v[2 * q + 1] = *reinterpret_cast<const float4*>(next + (2 * q + 1) * dim + lane_off);
         }
+    };
+    auto finish = [&](const Pieces& out, int buf_off) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            *reinterpret_cast<halfx8*>(st_dst + buf_off + 32 * j * kFRowW) = hi[j];
-            *reinterpret_cast<halfx8*>(st_dst + buf_off + kFPlane + 32 * j * kFRowW) = lo[j];
+            *reinterpret_cast<halfx8*>(st_dst + buf_off + 32 * j * kFRowW) = out.hi[j].all;
+            *reinterpret_cast<halfx8*>(st_dst + buf_off + kFPlane + 32 * j * kFRowW) = out.lo[j].all;
         }
     };
 
@@ -443,43 +476,27 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
             for (int k = 0; k < 16; k++) acc[p][q][k] = 0.f;
 
     // matrix lanes: LDS rows 64 (wave / 2) + 32 p + m of dy, 64 (wave % 2) + 32 q + m of x; 16-byte piece 2 step + g,
-    // swizzled with (row >> 2) & 3 = (m >> 2) & 3
-    const int sw = (m >> 2) & 3;
+    // swizzled
+    const int sw = swizzle(m);
     const unsigned char* a_lds = lds + ((wave >> 1) * 64 + m) * kFRowW;
     const unsigned char* b_lds = lds + 2 * kFPlane + ((wave & 1) * 64 + m) * kFRowW;
-    auto multiply = [&](int buf_off) {
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            const int piece = buf_off + 16 * ((2 * s + g) ^ sw);
-            halfx8 ah[2], al[2], bh[2], bl[2];
-#pragma unroll
-            for (int p = 0; p < 2; p++) {
-                ah[p] = *reinterpret_cast<const halfx8*>(a_lds + piece + 32 * p * kFRowW);
-                al[p] = *reinterpret_cast<const halfx8*>(a_lds + piece + kFPlane + 32 * p * kFRowW);
-                bh[p] = *reinterpret_cast<const halfx8*>(b_lds + piece + 32 * p * kFRowW);
-                bl[p] = *reinterpret_cast<const halfx8*>(b_lds + piece + kFPlane + 32 * p * kFRowW);
-            }
-#pragma unroll
-            for (int p = 0; p < 2; p++)
-#pragma unroll
-                for (int q = 0; q < 2; q++) {
-                    // small terms first
-                    acc[p][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[p], bh[q], acc[p][q], 0, 0, 0);
-                    acc[p][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[p], bl[q], acc[p][q], 0, 0, 0);
-                    acc[p][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[p], bh[q], acc[p][q], 0, 0, 0);
-                }
-        }
+    halfx8 ah[2], al[2], bh[2], bl[2];
+    auto read_a = [&](int p, int s, int buf_off) {
+        const unsigned char* at = a_lds + buf_off + 16 * ((2 * s + g) ^ sw) + 32 * p * kFRowW;
+        ah[p] = *reinterpret_cast<const halfx8*>(at);
+        al[p] = *reinterpret_cast<const halfx8*>(at + kFPlane);
+    };
+    auto read_b = [&](int q, int s, int buf_off) {
+        const unsigned char* at = b_lds + buf_off + 16 * ((2 * s + g) ^ sw) + 32 * q * kFRowW;
+        bh[q] = *reinterpret_cast<const halfx8*>(at);
+        bl[q] = *reinterpret_cast<const halfx8*>(at + kFPlane);
+    };
+    auto product = [&](int p, int q) {                     // small terms first
+        acc[p][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[p], bh[q], acc[p][q], 0, 0, 0);
+        acc[p][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[p], bl[q], acc[p][q], 0, 0, 0);
+        acc[p][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[p], bh[q], acc[p][q], 0, 0, 0);
     };
 
-    // a stage is multiplied out of one buffer while the next one is split into the other and the loads of the one
-    // after that are on their way
-    // (stages past the slice are fetched and stored like the others, scaled by zero and never multiplied: the loop
-    // body has no branch, and the splitting of one stage can be issued between the matrix instructions of another)
-    fetch(r_lo);
-    set_scales();                                          // (the first stage is on its way meanwhile)
-    store(r_lo, 0);
-    fetch(r_lo + kFRows);
-    __syncthreads();
     // The matrix instructions accumulate runs of kFRun rows; the runs are added in a second set of registers: the
     // rounding error of an fp32 sum grows with its length, and a slice of 50 000 rows in one chain was 1.7 times
     // less accurate than the same sum in chunks.
@@ -490,29 +507,56 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int q = 0; q < 2; q++)
 #pragma unroll
             for (int k = 0; k < 16; k++) total[p][q][k] = 0.f;
-    int buf_off = 0;
-    for (long r = r_lo; r < r_hi;) {
-        const long run_hi = r + kFRun < r_hi ? r + kFRun : r_hi;
-        for (; r < run_hi; r += kFRows) {
-            multiply(buf_off);
-            buf_off ^= kFBuf;
-            store(r + kFRows, buf_off);
-            fetch(r + 2 * kFRows);
+    // A stage is multiplied out of one buffer while the next one is split into the other and the loads of the one
+    // after that are on their way; three matrix instructions and a part of the splitting in turn, in this order (left to itself the
+    // compiler multiplies first and splits then, and every load is waited for as soon as it is sent).
+    // (stages past the slice are fetched and stored like the others, scaled by zero and never multiplied: the loop
+    // body has no branch)
+    auto walk = [&](auto sums) {
+        Pieces next;
 #pragma unroll
-            for (int k = 0; k < 24; k++) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);     // one matrix instruction,
-                __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);     // seven vector instructions in its shadow
+        for (int k = 0; k < 8; k++) split_part(k, next, r_lo, r_lo + kFRows, sums);
+        finish(next, 0);
+        __syncthreads();
+        int buf_off = 0;
+        for (long r = r_lo; r < r_hi;) {
+            const long run_hi = r + kFRun < r_hi ? r + kFRun : r_hi;
+            for (; r < run_hi; r += kFRows) {
+                read_a(0, 0, buf_off);
+                read_b(0, 0, buf_off);
+                read_b(1, 0, buf_off);
+                read_a(1, 0, buf_off);
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    split_part(k, next, r + kFRows, r + 2 * kFRows, sums);
+                    __builtin_amdgcn_sched_barrier(0);
+                    product(k >> 1 & 1, k & 1);
+                    if (k == 1) read_a(0, 1, buf_off);
+                    if (k == 2) read_b(0, 1, buf_off);
+                    if (k == 3) {
+                        read_b(1, 1, buf_off);
+                        read_a(1, 1, buf_off);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                buf_off ^= kFBuf;
+                finish(next, buf_off);
+                __syncthreads();
             }
-            __syncthreads();
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+#pragma unroll
+                for (int q = 0; q < 2; q++)
+#pragma unroll
+                    for (int k = 0; k < 16; k++) { total[p][q][k] += acc[p][q][k]; acc[p][q][k] = 0.f; }
         }
-#pragma unroll
-        for (int p = 0; p < 2; p++)
-#pragma unroll
-            for (int q = 0; q < 2; q++)
-#pragma unroll
-                for (int k = 0; k < 16; k++) { total[p][q][k] += acc[p][q][k]; acc[p][q][k] = 0.f; }
-    }
-    if (colsum_part != nullptr && blockIdx.y == 0) {                              // (uniform)
+    };
+    fetch(r_lo);
+    set_scales();                                          // (the first stage is on its way meanwhile)
+    if (sum_cols) walk(std::true_type{});
+    else walk(std::false_type{});
+    if (colsum_part != nullptr && i_tile == 0) {                              // (uniform)
         // the four row groups of a column quad, added in a fixed order
         float4* sums = reinterpret_cast<float4*>(lds);                             // [octet][cq]; the stage buffers are done with
         if (!stage_x) sums[octet * 32 + cq] = colsum;
@@ -521,14 +565,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
             const float4 s0 = sums[cq], s1 = sums[32 + cq], s2 = sums[64 + cq], s3 = sums[96 + cq];
             const int o = o_tile + 4 * cq;
             if (o < O)
-                *reinterpret_cast<float4*>(colsum_part + (long)blockIdx.z * O + o) =
+                *reinterpret_cast<float4*>(colsum_part + slice * O + o) =
                     make_float4((s0.x + s1.x) + (s2.x + s3.x), (s0.y + s1.y) + (s2.y + s3.y),
                                 (s0.z + s1.z) + (s2.z + s3.z), (s0.w + s1.w) + (s2.w + s3.w));
         }
     }
     // D[row][col]: col = lane % 32, row = 8 (k / 4) + 4 (lane / 32) + k % 4 for register k; LDS row 32 j + c / 4 of
     // an operand is column 4 (c / 4) + j of the tile
-    float* plane = part + (long)blockIdx.z * O * I;
+    float* plane = part + slice * O * I;
 #pragma unroll
     for (int p = 0; p < 2; p++)
 #pragma unroll
@@ -670,7 +714,9 @@ static int wgrad_f16x2(const float* dy, const float* x, const float* dy_bound, l
                            scan[1]);
     const float* dy_parts = (dy_bound && n_dy_bound <= kDirectBounds) ? dy_bound : maxima;
     const float* x_parts = (groups == 1 && x_bound && n_x_bound <= kDirectBounds) ? x_bound : maxima + kFParts;
-    dim3 grid((unsigned)ceil_div(dim_out, kFTile), (unsigned)ceil_div(dim_in, kFTile), (unsigned)splits), block(256);
+    const long items = ceil_div(dim_out, kFTile) * ceil_div(dim_in, kFTile) * splits;
+    MG_REQUIRE(items < (1L << 31) - 8, "mg_tensor_linear_wgrad_f16x2: grid too large");
+    dim3 grid((unsigned)(8 * ceil_div(items, 8))), block(256);
     hipLaunchKernelGGL(wgrad_f16x2_kernel, grid, block, 0, st, dy, x, dy_parts, na, x_parts, nb, dim_in / groups, rows, dim_in,
                        dim_out, rpb, part, colsum_part, bias_rows);
     const long n_sum = n + (db ? dim_out : 0);

@@ -582,6 +582,20 @@ def test_weight_gradient_split_fp16(ops, rows, dim_in, dim_out, bounds):
     assert not torch.equal(plain, got)          # (another kernel, another summation order)
 
 
+@pytest.mark.parametrize("rows, dim_in, dim_out", [(4096, 4, 4), (4097, 260, 132), (4127, 132, 388), (5000, 640, 128), (70001, 36, 260)])
+def test_wgrad_slices_and_tiles_over_the_chip(ops, rows, dim_in, dim_out):
+    """One tile and several, as many (slice, tile) pairs as no eighth of them is whole, a last stage that overlaps the one before: against
+    float64, the weights' gradient in its 2-norm (sums of runs of 256 rows: 2^-22 a product, random) and the bias row sums."""
+    g = torch.Generator().manual_seed(rows)
+    dy, x = torch.randn(rows, dim_out, generator=g).cuda(), torch.randn(rows, dim_in, generator=g).cuda()
+    dW, db = ops.tensor_linear_wgrad(0, dy, x, want_bias=True)
+    ref = dy.double().t() @ x.double()
+    assert float((dW.double() - ref).norm()) <= 1e-6 * float(ref.norm())
+    assert float((db.double() - dy.double().sum(0)).abs().max()) <= 2.0 ** -24 * rows ** 0.5 * 64
+    assert torch.equal(ops.tensor_linear_wgrad(0, dy, x), dW)
+
+
+
 def test_weight_gradient_at_the_edge_count_of_configs2(ops):
     """The split-fp16 weight gradient at the size training runs it at (1592454 edge rows, 512 x 512): against float64
     accumulated over row chunks on the device, with the error of torch's own fp32 product of the same operands as
