@@ -917,6 +917,11 @@ int mg_group_norm(int mode, const float* x, long x_stride, const float* mul, lon
                   int batch, int nodes, int chan, int groups, int comps, float eps,
                   const float* gamma, const float* beta, const float* add, long add_stride,
                   const float* res, void* scratch, float* out, mg_stream_t stream);
+/* Gradients of mode 0 for dense x and dy (batch, nodes, chan, comps), nothing added: dx like x, dgamma (chan).  scratch: what the
+ * forward call of this x left there. */
+int mg_tensor_norm_grad_workspace_bytes(int batch, int chan, int groups, int comps, size_t* bytes /* host */);
+int mg_tensor_norm_grad(const float* dy, const float* x, int batch, int nodes, int chan, int groups, int comps, float eps,
+                        const float* gamma, const void* scratch, void* workspace, float* dx, float* dgamma, mg_stream_t stream);
 /* tens_sigmoid (managan/tensor_products.py:167-182): x / sqrt(1 + sum_comp x^2) per (row, chan). */
 int mg_tens_sigmoid(int inds, const float* x, long rows_times_chan, float* out, mg_stream_t stream);
 /* kind 1: sq_radial_encode(normed_sq_dist(r, rmax), n) (archs/diffuser_atoms14.py:32-48);

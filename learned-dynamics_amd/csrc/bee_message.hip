@@ -69,19 +69,19 @@ __global__ void __launch_bounds__(256) bee_geometry_kernel(const float* __restri
     const float d = sqrtf(x * x + y * y + z * z);
     const float zz = d / r0;
     const double zd = (double)zz;
-    const float cut = fmaxf(1.0f - zz, 0.0f);
+    const double cut = zd < 1.0 ? 1.0 - zd : 0.0;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         double acc = jac.a[i][8];
 #pragma unroll
         for (int j = 7; j >= 0; j--) acc = acc * zd + jac.a[i][j];
-        enc[8 * e + i] = (float)(acc * (double)cut);
+        enc[8 * e + i] = (float)(acc * cut);
     }
     const float sx = x * scale, sy = y * scale, sz = z * scale;
-    const float inv = 1.0f / sqrtf(1.0f + (sx * sx + sy * sy + sz * sz));
-    rhat[3 * e] = sx * inv;
-    rhat[3 * e + 1] = sy * inv;
-    rhat[3 * e + 2] = sz * inv;
+    const float len = sqrtf(1.0f + (sx * sx + sy * sy + sz * sz));
+    rhat[3 * e] = sx / len;
+    rhat[3 * e + 1] = sy / len;
+    rhat[3 * e + 2] = sz / len;
 }
 
 // max over the wave of non-negative values (NaN counts as zero), valid in lane 63: six cross-lane VALU operations (shifts within

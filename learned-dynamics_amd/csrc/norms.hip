@@ -4,7 +4,7 @@
 // the encodings, edge-sized) arrays; the norms need one box-wide reduction each.
 //
 // Reductions are deterministic: workgroup partials in a caller-provided scratch
-// array (fp64), folded in a fixed order by the apply kernel.
+// array (fp64), folded in a fixed order by the apply kernels.
 #include "common.hpp"
 
 namespace mg {
@@ -76,27 +76,22 @@ __global__ void __launch_bounds__(256) group_stats_kernel(const float* __restric
     }
 }
 
-// fold the kChunks partials of every (box, group) in a fixed order and derive what the apply kernel uses:
-// partial[bg*kChunks*2 + {0,1}] <- totals, + 2 <- the mean that is subtracted (0 for the tensor norm),
-// + 3 <- the denominator sqrt(eps + variance or mean square); both rounded to float as the apply kernel takes them
-__global__ void group_finalize_kernel(double* __restrict__ partial, int n_bg, double count, int mode, float eps) {
-    const int bg = blockIdx.x * blockDim.x + threadIdx.x;
-    if (bg >= n_bg) return;
-    double* p = partial + (long)bg * kChunks * 2;
-    double s = 0.0, ss = 0.0;
-    for (int k = 0; k < kChunks; k++) { s += p[2 * k]; ss += p[2 * k + 1]; }
-    p[0] = s;
-    p[1] = ss;
-    if (mode == 0) {
-        p[2] = 0.0;
-        p[3] = (double)sqrtf(eps + (float)(ss / count));          // mean over nodes, group channels of sum_comp v^2
-    } else {
-        const double mean = s / count;
-        double var = ss / count - mean * mean;
-        var = var > 0.0 ? var : 0.0;
-        p[2] = (double)(float)mean;
-        p[3] = (double)sqrtf(eps + (float)var);
+// The kChunks partials of a (box, group), folded in a fixed order by a wave: in every lane .x the mean that is subtracted (0 for the
+// tensor norm), .y the denominator sqrt(eps + variance or mean square), both as the apply kernels take them
+__device__ __forceinline__ float2 fold_group(const double* __restrict__ partial, long bg, double count, int mode, float eps) {
+    static_assert(kChunks == kWave, "a lane to a partial sum");
+    const double* p = partial + (bg * kChunks + (threadIdx.x & (kWave - 1))) * 2;
+    double s = p[0], ss = p[1];
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) {
+        s += __shfl_xor(s, d);
+        ss += __shfl_xor(ss, d);
     }
+    if (mode == 0) return make_float2(0.f, sqrtf(eps + (float)(ss / count)));   // mean over nodes, group channels of sum_comp v^2
+    const double mean = s / count;
+    double var = ss / count - mean * mean;
+    var = var > 0.0 ? var : 0.0;
+    return make_float2((float)mean, sqrtf(eps + (float)var));
 }
 
 // mode 0 (TensGroupNorm): y = gamma[c] * v / sqrt(eps + mean(sum_comp v^2))
@@ -104,31 +99,122 @@ __global__ void group_finalize_kernel(double* __restrict__ partial, int n_bg, do
 // then y += add (optional, add_stride) and y += res (optional, same layout as out).
 // A thread keeps one (channel, component) position k = c*T + comp of the rows of box blockIdx.z and walks over
 // nodes: channel, group, gamma, beta and the group's statistics are fixed per thread, consecutive threads touch
-// consecutive floats.
+// consecutive floats.  A workgroup folds the partial sums of the groups that its positions belong to by itself (a launch for it took
+// 3 us on one system and 5 on 32 of them; each node array had one).
 __global__ void __launch_bounds__(256) group_apply_kernel(const float* __restrict__ x, long x_stride,
                                                           const float* __restrict__ mul, long mul_stride,
                                                           const double* __restrict__ partial, int N, int chan,
-                                                          int groups, int T, int mode,
+                                                          int groups, int T, int mode, float eps,
                                                           const float* __restrict__ gamma, const float* __restrict__ beta,
                                                           const float* __restrict__ add, long add_stride,
                                                           const float* __restrict__ res, float* __restrict__ out) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int CT = chan * T;
-    if (k >= CT) return;
-    const int b = blockIdx.z;
-    const int c = k / T, g = c / (chan / groups);
-    const double* p = partial + ((long)(b * groups + g) * kChunks) * 2;
-    const float mean = (float)p[2], denom = (float)p[3];
-    const float ga = gamma[c], be = mode == 0 ? 0.f : beta[c];
+    __shared__ float2 stats[256];                                  // (a position a thread: no more groups than that)
+    const int CT = chan * T, b = blockIdx.z, per = chan / groups * T;
+    const int k_first = blockIdx.x * blockDim.x, k = k_first + (int)threadIdx.x;
+    const int k_last = k_first + (int)blockDim.x < CT ? k_first + (int)blockDim.x - 1 : CT - 1, g_first = k_first / per;
+    const bool live = k < CT;
     const long x_row = x_stride * T, m_row = mul_stride * T, a_row = add_stride * T;
+    constexpr int kAhead = 4;                                      // nodes at a time; the first ones are on their way during the fold
+    float v[kAhead], plus[kAhead];
+    auto fetch = [&](int i) {
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) {
+            const int node = i + u * (int)gridDim.y;
+            const long row = (long)b * N + (node < N ? node : N - 1);
+            v[u] = live ? x[row * x_row + k] : 0.f;
+            if (mul && live) v[u] *= mul[row * m_row + k];
+            plus[u] = add && live ? add[row * a_row + k] : 0.f;
+            if (res && live) plus[u] += res[row * CT + k];
+        }
+    };
+    fetch(blockIdx.y);
+    for (int g = g_first + (int)(threadIdx.x / kWave); g <= k_last / per; g += (int)(blockDim.x / kWave)) {
+        const float2 f = fold_group(partial, (long)b * groups + g, (double)N * (chan / groups), mode, eps);
+        if ((threadIdx.x & (kWave - 1)) == 0) stats[g - g_first] = f;
+    }
+    __syncthreads();
+    if (!live) return;
+    const int c = k / T;
+    const float mean = stats[k / per - g_first].x, denom = stats[k / per - g_first].y;
+    const float ga = gamma[c], be = mode == 0 ? 0.f : beta[c];
+    for (int i = blockIdx.y; i < N; i += kAhead * (int)gridDim.y) {
+        if (i != (int)blockIdx.y) fetch(i);
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) {
+            const int node = i + u * (int)gridDim.y;
+            const float y = mode == 0 ? ga * (v[u] / denom) : be + ga * ((v[u] - mean) / denom);
+            if (node < N) out[((long)b * N + node) * CT + k] = y + plus[u];
+        }
+    }
+}
+
+// Gradient of the tensor norm y = gamma x / s, s = sqrt(eps + mean x^2) over a (box, group):
+//     dgamma[c] = sum dy x / s,   dx = gamma dy / s - x D / (s^3 count),   D = sum over the group of gamma dy x.
+// One pass sums dy x per channel position over chunks of a box's nodes, a second folds them group by group, a third forms dx:
+// 8192 nodes of 256 channels 21 us where a dozen of torch's passes took 130.  Both sums in fp64.
+// sums: [b][k][chunk]
+__global__ void __launch_bounds__(256) tensor_norm_grad_sums_kernel(const float* __restrict__ dy, const float* __restrict__ x, int N,
+                                                                    int CT, double* __restrict__ sums) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.z, chunk = blockIdx.y;
+    if (k >= CT) return;
+    const int per = (N + kChunks - 1) / kChunks, lo = chunk * per, hi = lo + per < N ? lo + per : N;
+    const long at = (long)b * N * CT + k;
+    double sum = 0.0;
+    int i = lo;
+    for (; i + 4 <= hi; i += 4) {                                  // (eight loads on their way)
+        float g[4], v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            g[u] = dy[at + (long)(i + u) * CT];
+            v[u] = x[at + (long)(i + u) * CT];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) sum += (double)g[u] * v[u];
+    }
+    for (; i < hi; i++) sum += (double)dy[at + (long)i * CT] * x[at + (long)i * CT];
+    sums[((long)b * CT + k) * kChunks + chunk] = sum;
+}
+
+// A workgroup to a (group, box).  coef[b groups + g] = (1 / s, D / (s^3 count)); of_box[b chan + c] = sum over the box of dy x / s
+__global__ void __launch_bounds__(256) tensor_norm_grad_fold_kernel(const double* __restrict__ sums, const double* __restrict__ partial,
+                                                                    const float* __restrict__ gamma, int N, int chan, int groups, int T,
+                                                                    float eps, float2* __restrict__ coef, double* __restrict__ of_box) {
+    __shared__ double of_wave[4];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int g = blockIdx.x, b = blockIdx.y, cg = chan / groups;
+    const double count = (double)N * cg, s = (double)fold_group(partial, (long)b * groups + g, count, 0, eps).y;
+    double d = 0.0;
+    for (int c = g * cg + wave; c < (g + 1) * cg; c += 4) {
+        double q = 0.0;
+        for (int t = 0; t < T; t++) q += sums[((long)b * chan * T + (long)c * T + t) * kChunks + lane];
+#pragma unroll
+        for (int e = kWave / 2; e > 0; e >>= 1) q += __shfl_xor(q, e);
+        d += (double)gamma[c] * q;
+        if (lane == 0) of_box[(long)b * chan + c] = q / s;
+    }
+    if (lane == 0) of_wave[wave] = d;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        coef[b * groups + g] = make_float2((float)(1.0 / s), (float)((of_wave[0] + of_wave[1] + of_wave[2] + of_wave[3]) / (s * s * s * count)));
+}
+
+// (the first workgroups also add up dgamma over the boxes)
+__global__ void __launch_bounds__(256) tensor_norm_grad_apply_kernel(const float* __restrict__ dy, const float* __restrict__ x, int batch,
+                                                                     int N, int chan, int groups, int T, const float* __restrict__ gamma,
+                                                                     const float2* __restrict__ coef, const double* __restrict__ of_box,
+                                                                     float* __restrict__ dx, float* __restrict__ dgamma) {
+    const int CT = chan * T, k = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.z;
+    if (k >= CT) return;
+    const float2 f = coef[b * groups + k / T / (chan / groups)];
+    const float scale = gamma[k / T] * f.x;
     for (int i = blockIdx.y; i < N; i += gridDim.y) {
-        const long row = (long)b * N + i;
-        float v = x[row * x_row + k];
-        if (mul) v *= mul[row * m_row + k];
-        float y = mode == 0 ? ga * (v / denom) : be + ga * ((v - mean) / denom);
-        if (add) y += add[row * a_row + k];
-        if (res) y += res[row * CT + k];
-        out[row * CT + k] = y;
+        const long at = ((long)b * N + i) * CT + k;
+        dx[at] = scale * dy[at] - f.y * x[at];
+    }
+    if (blockIdx.y == 0 && b == 0 && k % T == 0) {
+        double sum = 0.0;
+        for (int j = 0; j < batch; j++) sum += of_box[(long)j * chan + k / T];
+        dgamma[k / T] = (float)sum;
     }
 }
 
@@ -244,6 +330,17 @@ int mg_group_norm_scratch_bytes(int batch, int groups, size_t* bytes) {
     return MG_OK;
 }
 
+// Positions across, nodes of a box down: four nodes a thread, which it has on their way at once, and more where that is beyond 4096
+// workgroups, each of which folds by itself (2048 nodes of 256 channels 6.3 us, 8.4 at one node a thread, 7.4 in two launches; 65 536
+// 45 us in 4096 workgroups, 49 in 8192, 63 in 1024, 49 in two launches of 8192; 16 336 12.5, 15.5 in two)
+static dim3 apply_grid(int batch, int nodes, int CT, int* threads) {
+    *threads = CT >= 256 ? 256 : (int)ceil_div(CT, kWave) * kWave;
+    const long kx = ceil_div(CT, *threads), most = ceil_div(4096L, kx * batch);
+    long ny = ceil_div(nodes, 4);
+    ny = ny > most ? most : ny;
+    return dim3((unsigned)kx, (unsigned)ny, (unsigned)batch);
+}
+
 int mg_group_norm(int mode, const float* x, long x_stride, const float* mul, long mul_stride, int batch, int nodes,
                   int chan, int groups, int comps, float eps, const float* gamma, const float* beta, const float* add,
                   long add_stride, const float* res, void* scratch, float* out, mg_stream_t stream) {
@@ -258,17 +355,39 @@ int mg_group_norm(int mode, const float* x, long x_stride, const float* mul, lon
     hipStream_t st = (hipStream_t)stream;
     hipLaunchKernelGGL(group_stats_kernel, dim3((unsigned)(batch * groups), kChunks), dim3(256), 0, st, x, x_stride, mul,
                        mul_stride, nodes, chan, groups, comps, static_cast<double*>(scratch));
-    hipLaunchKernelGGL(group_finalize_kernel, dim3((unsigned)ceil_div((long)batch * groups, 64)), dim3(64), 0, st,
-                       static_cast<double*>(scratch), batch * groups, (double)nodes * (chan / groups), mode, eps);
-    const int CT = chan * comps;
-    const int threads = CT >= 256 ? 256 : (int)ceil_div(CT, kWave) * kWave;
-    const long kx = ceil_div(CT, threads);
-    long ny = ceil_div(8192L, kx * batch);                      // about 8192 workgroups, each thread a few nodes
-    ny = ny > nodes ? nodes : (ny < 1 ? 1 : ny);
-    hipLaunchKernelGGL(group_apply_kernel, dim3((unsigned)kx, (unsigned)ny, (unsigned)batch), dim3(threads), 0, st, x,
-                       x_stride, mul, mul_stride, static_cast<const double*>(scratch), nodes, chan, groups, comps, mode,
+    int threads;
+    const dim3 grid = apply_grid(batch, nodes, chan * comps, &threads);
+    hipLaunchKernelGGL(group_apply_kernel, grid, dim3(threads), 0, st, x,
+                       x_stride, mul, mul_stride, static_cast<const double*>(scratch), nodes, chan, groups, comps, mode, eps,
                        gamma, beta, add, add_stride, res, out);
     return check_launch("mg_group_norm");
+}
+
+int mg_tensor_norm_grad_workspace_bytes(int batch, int chan, int groups, int comps, size_t* bytes) {
+    MG_REQUIRE(bytes && batch >= 0 && chan >= 0 && groups >= 0 && comps >= 0, "mg_tensor_norm_grad_workspace_bytes: bad argument");
+    *bytes = (size_t)batch * chan * (comps * kChunks + 1) * sizeof(double) + (size_t)batch * groups * sizeof(float2);
+    return MG_OK;
+}
+
+int mg_tensor_norm_grad(const float* dy, const float* x, int batch, int nodes, int chan, int groups, int comps, float eps,
+                        const float* gamma, const void* scratch, void* workspace, float* dx, float* dgamma, mg_stream_t stream) {
+    MG_REQUIRE(batch >= 0 && nodes >= 0 && chan >= 0 && groups > 0 && chan % groups == 0, "mg_tensor_norm_grad: bad sizes");
+    MG_REQUIRE(comps == 1 || comps == 3 || comps == 9, "mg_tensor_norm_grad: comps must be 1, 3 or 9");
+    MG_REQUIRE(batch > 0 && nodes > 0 && chan > 0, "mg_tensor_norm_grad: nothing to differentiate");
+    MG_REQUIRE(dy && x && gamma && scratch && workspace && dx && dgamma, "mg_tensor_norm_grad: null pointer");
+    MG_REQUIRE(batch <= 65535 && (long)chan * comps <= 0x7fffffffL, "mg_tensor_norm_grad: more than 65535 boxes");
+    hipStream_t st = (hipStream_t)stream;
+    const int CT = chan * comps;
+    double *sums = static_cast<double*>(workspace), *of_box = sums + (long)batch * CT * kChunks;
+    float2* coef = reinterpret_cast<float2*>(of_box + (long)batch * chan);
+    int threads;
+    const dim3 grid = apply_grid(batch, nodes, CT, &threads);
+    hipLaunchKernelGGL(tensor_norm_grad_sums_kernel, dim3(grid.x, kChunks, grid.z), dim3(threads), 0, st, dy, x, nodes, CT, sums);
+    hipLaunchKernelGGL(tensor_norm_grad_fold_kernel, dim3((unsigned)groups, (unsigned)batch), dim3(256), 0, st, sums,
+                       static_cast<const double*>(scratch), gamma, nodes, chan, groups, comps, eps, coef, of_box);
+    hipLaunchKernelGGL(tensor_norm_grad_apply_kernel, grid, dim3(threads), 0, st, dy, x, batch, nodes, chan, groups, comps, gamma, coef, of_box,
+                       dx, dgamma);
+    return check_launch("mg_tensor_norm_grad");
 }
 
 int mg_tens_sigmoid(int inds, const float* x, long rows_times_chan, float* out, mg_stream_t stream) {

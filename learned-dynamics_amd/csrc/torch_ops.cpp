@@ -631,6 +631,38 @@ std::tuple<at::Tensor, at::Tensor> painn_update(const at::Tensor& x_a, const at:
     return {out_a, out_v};
 }
 
+// TensGroupNorm.forward of x (batch, nodes, chan, ..) and the sums that its adjoint reads again
+std::tuple<at::Tensor, at::Tensor> tens_norm_fwd(const at::Tensor& x, const at::Tensor& gamma, int groups, double eps) {
+    check_input(x, "x");
+    check_input(gamma, "gamma");
+    TORCH_CHECK(x.dim() >= 3 && x.dim() <= 5 && gamma.numel() == x.size(2), "x must have shape (batch, nodes, chan, (3,)^inds)");
+    const int64_t B = x.size(0), N = x.size(1), C = x.size(2), T = C * N * B ? x.numel() / (B * N * C) : 1;
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    size_t n = 0;
+    check(mg_group_norm_scratch_bytes((int)B, groups, &n));
+    at::Tensor scratch = bytes_like(x, std::max<size_t>(n, 8)), y = floats(x, x.sizes());
+    check(mg_group_norm(0, fp(x), C, nullptr, 0, (int)B, (int)N, (int)C, groups, (int)T, (float)eps, fp(gamma), nullptr, nullptr, 0, nullptr,
+                        scratch.data_ptr(), fp(y), stream_of(x)));
+    return {y, scratch};
+}
+std::tuple<at::Tensor, at::Tensor> tens_norm_bwd(const at::Tensor& dy, const at::Tensor& x, const at::Tensor& gamma, const at::Tensor& scratch,
+                                                 int groups, double eps) {
+    check_input(dy, "dy");
+    check_input(x, "x");
+    check_input(gamma, "gamma");
+    TORCH_CHECK(x.dim() >= 3 && x.dim() <= 5 && dy.sizes() == x.sizes() && gamma.numel() == x.size(2) && x.numel() > 0, "tens_norm_bwd: sizes");
+    const int64_t B = x.size(0), N = x.size(1), C = x.size(2), T = x.numel() / (B * N * C);
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    size_t n = 0, kept = 0;
+    check(mg_tensor_norm_grad_workspace_bytes((int)B, (int)C, groups, (int)T, &n));
+    check(mg_group_norm_scratch_bytes((int)B, groups, &kept));
+    TORCH_CHECK(scratch.is_cuda() && scratch.is_contiguous() && (size_t)scratch.nbytes() >= kept, "tens_norm_bwd: the sums of the forward pass");
+    at::Tensor ws = bytes_like(x, n), dx = floats(x, x.sizes()), dgamma = floats(x, gamma.sizes());
+    check(mg_tensor_norm_grad(fp(dy), fp(x), (int)B, (int)N, (int)C, groups, (int)T, (float)eps, fp(gamma), scratch.data_ptr(), ws.data_ptr(),
+                              fp(dx), fp(dgamma), stream_of(x)));
+    return {dx, dgamma};
+}
+
 struct MessageArgs {
     const at::Tensor &row_ptr, &dst, &r_ij, &x_a, &x_v;
     int64_t B, N, n, rows, E;
@@ -1581,6 +1613,8 @@ void register_ops(pybind11::module_& m) {
     m.def("row_linears_bwd", &row_linears_bwd);
     m.def("silu_order", &silu_order);
     m.def("linear_chain", &linear_chain);
+    m.def("tens_norm_fwd", &tens_norm_fwd);
+    m.def("tens_norm_bwd", &tens_norm_bwd);
     m.def("filter_grid", &filter_grid);
     m.def("filter_grids", &filter_grids);
     m.def("mlp_takes_rows", &mlp_takes_rows);

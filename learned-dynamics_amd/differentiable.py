@@ -403,12 +403,45 @@ def scal_group_norm(gn, x, gamma=None, beta=None):
     return add(mul((sh / torch.sqrt(add(var, gn.epsilon))).reshape(B, N, chan), gamma), beta)
 
 
+def _tens_norm_plain(x, gamma, groups, eps):
+    """managan/tensor_products.py:215-232"""
+    B, N = x.shape[:2]
+    xg = x.reshape(B, N, groups, -1, math.prod(x.shape[3:]))
+    m2 = (xg ** 2).sum(-1, keepdim=True).mean([1, 3], keepdim=True)
+    return mul((xg / torch.sqrt(add(m2, eps))).reshape(x.shape), gamma)
+
+
+class _TensNorm(torch.autograd.Function):
+    """TensGroupNorm: two passes each way and one between them, sums in float64."""
+
+    @staticmethod
+    def forward(ctx, x, gamma, groups, eps):
+        y, sums = ops.tens_norm_fwd(x, gamma, groups, eps)
+        ctx.save_for_backward(x, gamma, sums)
+        ctx.groups, ctx.eps = groups, eps
+        ctx.set_materialize_grads(False)
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, gamma, sums = ctx.saved_tensors
+        need = ctx.needs_input_grad[:2]
+        if dy is None:
+            return None, None, None, None
+        pieces = _gradients_in_pieces(lambda x, g: (_tens_norm_plain(x, g, ctx.groups, ctx.eps),), (x, gamma), need, (dy,))
+        if pieces is not None:
+            return pieces + (None, None)
+        dx, dgamma = ops.tens_norm_bwd(dy.contiguous(), x, gamma, sums, ctx.groups, ctx.eps)
+        return dx if need[0] else None, dgamma if need[1] else None, None, None
+
+
 def tens_group_norm(gn, x):
     """managan/tensor_products.py:215-232"""
-    B, N, chan = x.shape[:3]
-    xg = x.reshape(B, N, gn.groups, -1, 3 ** gn.inds)
-    m2 = (xg ** 2).sum(-1, keepdim=True).mean([1, 3], keepdim=True)
-    return mul((xg / torch.sqrt(add(m2, gn.epsilon))).reshape(x.shape), gn.gamma)
+    gamma = gn.gamma
+    fused = (x.is_cuda and x.dtype == gamma.dtype == torch.float32 and gamma.is_cuda and gamma.is_contiguous() and x.numel() > 0
+             and x.shape[0] <= 65535 and tuple(x.shape[2:]) == (gn.chan, *[3] * gn.inds)
+             and not has_tangent(x) and not has_tangent(gamma) and torch._C._functorch.peek_interpreter_stack() is None)
+    return _TensNorm.apply(x.contiguous(), gamma, gn.groups, gn.epsilon) if fused else _tens_norm_plain(x, gamma, gn.groups, gn.epsilon)
 
 
 def edge_vectors(graph, pos, box):
@@ -1221,9 +1254,11 @@ class _EdgeFilters(torch.autograd.Function):
 
 def bee_messages(msg, graph, r_ij, x_a, x_v, x_d):
     """archs/diffuser_atoms15.py:238-253"""
-    enc8 = radial_encode_8(r_ij, msg.r0)
+    if differentiated(r_ij) or not (r_ij.is_cuda and r_ij.dtype == torch.float32):
+        enc8, rh = radial_encode_8(r_ij, msg.r0), tens_sigmoid(1, mul(r_ij, 7. / msg.r0))
+    else:
+        enc8, rh = ops.bee_edge_geometry(r_ij.contiguous(), msg.r0)            # (two dozen of torch's passes over the edges)
     enc = linear(msg.lin_enc, enc8)
-    rh = tens_sigmoid(1, mul(r_ij, 7. / msg.r0))
     # The output linears of the vector and rank-2 channels have no bias and nothing nonlinear follows them before the
     # sum over edges, so they commute with it: the products are summed per node first and the ten linears run on N
     # rows, not E (the reference applies them per edge).  The scalar channel goes through an MLP per edge.

@@ -2332,6 +2332,11 @@ def group_norm(mode, x, groups, gamma, beta=None, eps=1e-5, mul=None, add=None, 
     return out
 
 
+# TensGroupNorm.forward with the sums that its adjoint reads, and the adjoint: (x (batch, nodes, chan, ..), gamma, groups, eps) -> (y,
+# sums); (dy, x, gamma, sums, groups, eps) -> (dx, dgamma)
+tens_norm_fwd, tens_norm_bwd = _ext.tens_norm_fwd, _ext.tens_norm_bwd
+
+
 def tens_sigmoid(inds, x):
     _check_input(x, "x")
     T = 3 ** inds
