@@ -320,19 +320,40 @@ __global__ void __launch_bounds__(256) grid_grad_finish_kernel(const float* __re
 }
 
 // ------------------------------------------------------------------------------------------------ stable sort by small keys
-// One pass of a stable radix sort on 9 bits: counts per (digit, chunk of 4096), their prefix sums per digit, and the scatter,
-// in which a wave ranks 64 elements at a time by comparing digits across lanes.  (torch.sort on these keys takes 10 launches:
-// 150 us for 1.6 M edges, 90 for 90 000; this takes 3.)
-constexpr int kDigits = 512, kDigitBits = 9, kSortChunk = 4096;
-__device__ __forceinline__ int digit_of(const int* keys, long i, int shift) { return (keys[i] >> shift) & (kDigits - 1); }
+// One pass of a stable radix sort on 9 bits: counts per (digit, chunk), their prefix sums per digit, and the scatter, in which a
+// wave ranks 64 elements at a time by comparing digits across lanes.  (torch.sort on these keys takes 10 launches: 150 us for
+// 1.6 M edges, 90 for 90 000; this takes 3.)
+// What bounds it is the chain within a workgroup, not the bytes: a thread therefore loads all PER of its keys at once and keeps them
+// for both loops, and a chunk (256 PER elements) is as short as leaves each compute unit a workgroup, down to two elements a thread.  One pass over
+// 78 000 keys: count 3.5, sums 4, scatter 5 us (chunks of 4096 read in the loops: 6-9, 4, 17); 8000 keys 5, 5, 5 (6-8, 5, 20);
+// 1.4 M keys 6, 5, 22 (8, 5, 29).
+constexpr int kDigits = 512, kDigitBits = 9;
+int sort_per_thread(long n) {
+    int per = 2;
+    while (per < 16 && n > 256L * 256 * per) per *= 2;
+    return per;
+}
+// the PER keys of a thread: element k of wave w is 64 (PER w + k) + lane of the chunk, so that a wave's elements are consecutive
+template <int PER>
+__device__ __forceinline__ long sort_element(int k) {
+    return ((long)blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 * PER) + 64 * k + (threadIdx.x & 63);
+}
 
+template <int PER>
 __global__ void __launch_bounds__(256) sort_count_kernel(const int* __restrict__ keys, long n, int shift, int chunks,
                                                          int* __restrict__ counts) {
     __shared__ int hist[kDigits];
+    int key[PER];
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+        const long i = sort_element<PER>(k);
+        key[k] = keys[min(i, n - 1)];
+    }
     for (int d = threadIdx.x; d < kDigits; d += 256) hist[d] = 0;
     __syncthreads();
-    const long lo = (long)blockIdx.x * kSortChunk, hi = min(lo + kSortChunk, n);
-    for (long i = lo + threadIdx.x; i < hi; i += 256) atomicAdd(&hist[digit_of(keys, i, shift)], 1);
+#pragma unroll
+    for (int k = 0; k < PER; k++)
+        if (sort_element<PER>(k) < n) atomicAdd(&hist[(key[k] >> shift) & (kDigits - 1)], 1);
     __syncthreads();
     for (int d = threadIdx.x; d < kDigits; d += 256) counts[(long)d * chunks + blockIdx.x] = hist[d];
 }
@@ -353,6 +374,7 @@ __global__ void __launch_bounds__(64) sort_prefix_kernel(int* __restrict__ count
     }
     if (threadIdx.x == 0) totals[blockIdx.x] = base;
 }
+template <int PER>
 __global__ void __launch_bounds__(256) sort_scatter_kernel(const int* __restrict__ keys, const int* __restrict__ values, long n,
                                                            int shift, int chunks, const int* __restrict__ counts,
                                                            const int* __restrict__ totals, int* __restrict__ keys_out,
@@ -360,6 +382,13 @@ __global__ void __launch_bounds__(256) sort_scatter_kernel(const int* __restrict
     __shared__ int at[4][kDigits];                            // next output position per wave and digit
     __shared__ int wave_sum[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int key[PER], value[PER];
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+        const long i = min(sort_element<PER>(k), n - 1);
+        key[k] = keys[i];
+        value[k] = values ? values[i] : (int)i;
+    }
     // exclusive prefix sums of the totals: two digits per thread
     {
         const int a = totals[2 * tid], b = totals[2 * tid + 1];
@@ -377,23 +406,20 @@ __global__ void __launch_bounds__(256) sort_scatter_kernel(const int* __restrict
         for (int w = 1; w < 4; w++) { at[w][2 * tid] = 0; at[w][2 * tid + 1] = 0; }
     }
     __syncthreads();
-    const long lo = (long)blockIdx.x * kSortChunk + (long)wave * (kSortChunk / 4);
-    const long hi = min(min(lo + kSortChunk / 4, ((long)blockIdx.x + 1) * kSortChunk), n);
     // how many of each digit the waves before this one hold
     if (wave < 3)
-        for (long i = lo + lane; i < hi; i += 64) {
-            const int d = digit_of(keys, i, shift);
-            for (int w = wave + 1; w < 4; w++) atomicAdd(&at[w][d], 1);
-        }
+#pragma unroll
+        for (int k = 0; k < PER; k++)
+            if (sort_element<PER>(k) < n)
+                for (int w = wave + 1; w < 4; w++) atomicAdd(&at[w][(key[k] >> shift) & (kDigits - 1)], 1);
     __syncthreads();
     for (int d = tid; d < kDigits; d += 256)
         for (int w = 1; w < 4; w++) at[w][d] += at[0][d];
     __syncthreads();
-    for (long i0 = lo; i0 < hi; i0 += 64) {
-        const long i = i0 + lane;
-        const bool live = i < hi;
-        const int key = live ? keys[i] : 0;
-        const int d = (key >> shift) & (kDigits - 1);
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+        const bool live = sort_element<PER>(k) < n;
+        const int d = (key[k] >> shift) & (kDigits - 1);
         unsigned long long same = __ballot(live);
 #pragma unroll
         for (int b = 0; b < kDigitBits; b++) {
@@ -409,8 +435,8 @@ __global__ void __launch_bounds__(256) sort_scatter_kernel(const int* __restrict
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
         if (live) {
-            values_out[pos] = values ? values[i] : (int)i;
-            if (keys_out) keys_out[pos] = key;
+            values_out[pos] = value[k];
+            if (keys_out) keys_out[pos] = key[k];
         }
     }
 }
@@ -530,7 +556,7 @@ int mg_painn_grid_table_grad(const int* order, const int* bucket_ptr, const int*
 
 int mg_sort_by_key_workspace_bytes(long count, size_t* bytes) {
     MG_REQUIRE(bytes && count >= 0, "mg_sort_by_key_workspace_bytes: bad argument");
-    *bytes = ((size_t)(ceil_div(count, kSortChunk) + 1) * kDigits + 3 * (size_t)count) * sizeof(int);
+    *bytes = ((size_t)(ceil_div(count, 256L * sort_per_thread(count)) + 1) * kDigits + 3 * (size_t)count) * sizeof(int);
     return MG_OK;
 }
 
@@ -544,7 +570,7 @@ int mg_sort_values_by_key(const int* keys, const int* values, long count, int ke
     if (count == 0) return MG_OK;
     MG_REQUIRE(keys && workspace && order && sorted_keys, "mg_sort_by_key: null pointer");
     hipStream_t st = (hipStream_t)stream;
-    const int chunks = (int)ceil_div(count, kSortChunk);
+    const int per = sort_per_thread(count), chunks = (int)ceil_div(count, 256L * per);
     int* counts = static_cast<int*>(workspace);
     int* totals = counts + (long)chunks * kDigits;
     int *spare_keys = totals + kDigits, *spare_values = spare_keys + count;
@@ -555,10 +581,18 @@ int mg_sort_values_by_key(const int* keys, const int* values, long count, int ke
         // the last pass ends in the caller's arrays
         const bool to_out = (passes - 1 - p) % 2 == 0;
         int *k_out = to_out ? sorted_keys : spare_keys, *v_out = to_out ? order : spare_values;
-        hipLaunchKernelGGL(sort_count_kernel, dim3(chunks), dim3(256), 0, st, k_in, count, kDigitBits * p, chunks, counts);
-        hipLaunchKernelGGL(sort_prefix_kernel, dim3(kDigits), dim3(64), 0, st, counts, chunks, totals);
-        hipLaunchKernelGGL(sort_scatter_kernel, dim3(chunks), dim3(256), 0, st, k_in, v_in, count, kDigitBits * p, chunks, counts,
-                           totals, k_out, v_out);
+        const auto pass = [&](auto count_kernel, auto scatter_kernel) {
+            hipLaunchKernelGGL(count_kernel, dim3(chunks), dim3(256), 0, st, k_in, count, kDigitBits * p, chunks, counts);
+            hipLaunchKernelGGL(sort_prefix_kernel, dim3(kDigits), dim3(64), 0, st, counts, chunks, totals);
+            hipLaunchKernelGGL(scatter_kernel, dim3(chunks), dim3(256), 0, st, k_in, v_in, count, kDigitBits * p, chunks,
+                               (const int*)counts, (const int*)totals, k_out, v_out);
+        };
+        switch (per) {
+            case 2: pass(sort_count_kernel<2>, sort_scatter_kernel<2>); break;
+            case 4: pass(sort_count_kernel<4>, sort_scatter_kernel<4>); break;
+            case 8: pass(sort_count_kernel<8>, sort_scatter_kernel<8>); break;
+            default: pass(sort_count_kernel<16>, sort_scatter_kernel<16>); break;
+        }
         k_in = k_out;
         v_in = v_out;
     }
