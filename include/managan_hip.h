@@ -697,6 +697,11 @@ int mg_painn_grid_node_grad(const int* row_ptr, const int* order, const int* src
                             const float* r_ij, const float* table, int table_rows, float period, float epsilon, const float* g_v,
                             const float* g_a, const float* actv, const float* v, int n, void* workspace, float* d_actv, float* d_v,
                             mg_stream_t stream);
+/* the same with the rows add_v (n_nodes, n, 3) added to d_v, unless NULL */
+int mg_painn_grid_node_add_grad(const int* row_ptr, const int* order, const int* src, const int* node_order, int n_nodes, long n_edges,
+                                const float* r_ij, const float* table, int table_rows, float period, float epsilon, const float* g_v,
+                                const float* g_a, const float* actv, const float* v, int n, void* workspace, const float* add_v,
+                                float* d_actv, float* d_v, mg_stream_t stream);
 /* row[e]: the grid row below an edge's length */
 int mg_painn_grid_rows(const float* r_ij, long n_edges, int table_rows, float period, int* row, mg_stream_t stream);
 /* The same with the edges of a graph (row_ptr over n_nodes sources) taken source by source in node_order: row and edge per position.
@@ -748,6 +753,17 @@ typedef struct mg_painn_combine_dual_grad {
 int mg_painn_combine_dual_bwd(const mg_painn_combine_dual* in, const int* row_ptr, const int* order, const float* g_v,
                               const float* g_v_t, const float* g_a, const float* g_a_t, const int* grad_row, long n_grad_rows,
                               const mg_painn_combine_dual_grad* grad, mg_stream_t stream);
+/* The same with rows added to the results: the layer's own input to the sums (x + message), and in the adjoint the gradients that
+ * reach that input past the message, to the gradients of v and v_t (v, v_t of `added`; its a, a_t are not read).  NULL: none. */
+typedef struct mg_painn_rows {
+    const float *a, *a_t, *v, *v_t;                /* (rows, n), (rows, n), (rows, n, 3), (rows, n, 3) */
+} mg_painn_rows;
+int mg_painn_combine_dual_add_fwd(const mg_painn_combine_dual* in, const int* node, const int* row_ptr, long n_out,
+                                  const mg_painn_rows* residual, float* out_v, float* out_v_t, float* out_a, float* out_a_t,
+                                  mg_stream_t stream);
+int mg_painn_combine_dual_add_bwd(const mg_painn_combine_dual* in, const int* row_ptr, const int* order, const float* g_v,
+                                  const float* g_v_t, const float* g_a, const float* g_a_t, const int* grad_row, long n_grad_rows,
+                                  const mg_painn_rows* added, const mg_painn_combine_dual_grad* grad, mg_stream_t stream);
 /* The update (archs/meanflow_painn8.py:63-75) around its MLP.  lrv (rows, 3, 3n): the maps l, r, v of x_v, component-major.
  * pre: ip = l . r, cat = [x_a, |r|].  post, with y = mlp(cat) (rows, 3n) and rows = batch x nodes:
  * out_a = groupnorm(ip y2) + y3, out_v = w / sqrt(|w|^2 + 1), w = v y1.  stats: 4 floats per box and group, written by post_fwd
@@ -765,6 +781,13 @@ int mg_painn_update_post_bwd(const float* lrv, const float* ip, const float* y, 
                              float* d_gamma, float* d_beta, mg_stream_t stream);
 int mg_painn_update_pre_bwd(const float* lrv, const float* g_ip, const float* g_cat, long rows, int n, int dual, float* g_lrv,
                             float* g_lrv_rowmax, float* g_xa, mg_stream_t stream);
+/* post_fwd with rows added to the results and the tangents' results apart, pre_bwd with rows (a, a_t of `added`) added to g_xa */
+int mg_painn_update_post_add_fwd(const float* lrv, const float* ip, const float* y, const float* gamma, const float* beta, int batch,
+                                 int nodes, int n, int groups, float eps, int dual, float* scratch, float* stats,
+                                 const mg_painn_rows* residual, float* out_a, float* out_a_t, float* out_v, float* out_v_t,
+                                 mg_stream_t stream);
+int mg_painn_update_pre_add_bwd(const float* lrv, const float* g_ip, const float* g_cat, long rows, int n, int dual, float* g_lrv,
+                                float* g_lrv_rowmax, const mg_painn_rows* added, float* g_xa, mg_stream_t stream);
 
 /* The first two layers of the radial MLP from the edge vectors (archs/meanflow_painn8.py:25-35 feeding :38-51):
  *   y[e] = SiLU(b2 + W2 SiLU(b1 + W1 radial_encode(r_ij[e], 16, rmax))),   y (E, hidden)

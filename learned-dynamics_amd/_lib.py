@@ -153,6 +153,11 @@ _SIGNATURES = {
     "mg_painn_edge_encode_fwd": [vp, vp, i64, i32, f32, f32, vp, vp, vp, vp, vp],
     "mg_painn_edge_encode_bwd": [vp, vp, i64, i32, f32, f32, vp, vp, vp, vp, vp, vp],
     "mg_painn_combine_dual_fwd": [vp, vp, vp, i64, vp, vp, vp, vp, vp],
+    "mg_painn_combine_dual_add_fwd": [vp, vp, vp, i64, vp, vp, vp, vp, vp, vp],
+    "mg_painn_combine_dual_add_bwd": [vp, vp, vp, vp, vp, vp, vp, vp, i64, vp, vp, vp],
+    "mg_painn_update_post_add_fwd": [vp, vp, vp, vp, vp, i32, i32, i32, i32, f32, i32, vp, vp, vp, vp, vp, vp, vp, vp],
+    "mg_painn_update_pre_add_bwd": [vp, vp, vp, i64, i32, i32, vp, vp, vp, vp, vp],
+    "mg_painn_grid_node_add_grad": [vp, vp, vp, vp, i32, i64, vp, vp, i32, f32, f32, vp, vp, vp, vp, i32, vp, vp, vp, vp, vp],
     "mg_painn_combine_dual_bwd": [vp, vp, vp, vp, vp, vp, vp, vp, i64, vp, vp],
     "mg_painn_update_pre_fwd": [vp, vp, vp, i64, i32, i32, vp, vp, vp, vp],
     "mg_painn_update_scratch_floats": [i32, i32, i32, i32, vp, vp],

@@ -292,6 +292,18 @@ __device__ __forceinline__ void st_unless_null(float* p, long off, const T& r) {
         for (int q = 0; q < V; q += 2) *reinterpret_cast<float2*>(p + off + q) = make_float2(r.f[q], r.f[q + 1]);
     }
 }
+template <int V>
+__device__ __forceinline__ Chans<V> plus(Chans<V> a, const Chans<V>& b) {
+#pragma unroll
+    for (int j = 0; j < V; j++) a.f[j] += b.f[j];
+    return a;
+}
+template <int V>
+__device__ __forceinline__ Vec3s<V> plus(Vec3s<V> a, const Vec3s<V>& b) {
+#pragma unroll
+    for (int j = 0; j < 3 * V; j++) a.f[j] += b.f[j];
+    return a;
+}
 template <int V> __device__ __forceinline__ Chans<V> ld_chans(const float* p, long off) { return ld_or_zero<V, Chans<V>>(p, off); }
 template <int V> __device__ __forceinline__ Vec3s<V> ld_vecs(const float* p, long off) { return ld_or_zero<3 * V, Vec3s<V>>(p, off); }
 __device__ __forceinline__ Vec3 ld3_or_zero(const float* p, long off) {
@@ -306,7 +318,7 @@ __device__ __forceinline__ long xcd_block() { return (long)(blockIdx.x & 7) * (g
 template <int V>
 __global__ void __launch_bounds__(256) combine_dual_fwd_kernel(CombineIn in, const int* __restrict__ node, long n_rows,
                                                                const int* __restrict__ row_ptr, long n_out, long E, int n,
-                                                               float* __restrict__ out_v, float* __restrict__ out_vt,
+                                                               mg_painn_rows res, float* __restrict__ out_v, float* __restrict__ out_vt,
                                                                float* __restrict__ out_a, float* __restrict__ out_at) {
     const int tpe = n / V;
     const long t = xcd_block() * 256 + threadIdx.x;
@@ -343,10 +355,10 @@ __global__ void __launch_bounds__(256) combine_dual_fwd_kernel(CombineIn in, con
             aat.f[j] += pt[3].f[j];
         }
     }
-    st_unless_null<3 * V>(out_v, (r * n + c) * 3, am);
-    st_unless_null<3 * V>(out_vt, (r * n + c) * 3, amt);
-    st_unless_null<V>(out_a, r * n + c, aa);
-    st_unless_null<V>(out_at, r * n + c, aat);
+    st_unless_null<3 * V>(out_v, (r * n + c) * 3, plus(am, ld_vecs<V>(res.v, (r * n + c) * 3)));
+    st_unless_null<3 * V>(out_vt, (r * n + c) * 3, plus(amt, ld_vecs<V>(res.v_t, (r * n + c) * 3)));
+    st_unless_null<V>(out_a, r * n + c, plus(aa, ld_chans<V>(res.a, r * n + c)));
+    st_unless_null<V>(out_at, r * n + c, plus(aat, ld_chans<V>(res.a_t, r * n + c)));
 }
 
 // Its adjoint, by destination row as painn_combine_bwd_rows_kernel: the gradients of actv and v (and of their tangents) are
@@ -360,7 +372,7 @@ __global__ void __launch_bounds__(256, 2) combine_dual_bwd_kernel(CombineIn in, 
                                                                   const float* __restrict__ gm, const float* __restrict__ gmt,
                                                                   const float* __restrict__ ga, const float* __restrict__ gat,
                                                                   const int* __restrict__ grad_row, long n_grad_rows, long E, int n,
-                                                                  CombineGrad out) {
+                                                                  CombineGrad out, mg_painn_rows add) {
     const int tpe = n / V;                                        // a power of two <= 64: a group never straddles waves
     const long t = xcd_block() * 256 + threadIdx.x;
     const long r_raw = t / tpe;
@@ -460,8 +472,8 @@ __global__ void __launch_bounds__(256, 2) combine_dual_bwd_kernel(CombineIn in, 
         st_unless_null<V>(out.actv, r * 4 * n + k * n + c, acc_a[k]);
         st_unless_null<V>(out.actv_t, r * 4 * n + k * n + c, acc_at[k]);
     }
-    st_unless_null<3 * V>(out.v, (r * n + c) * 3, acc_v);
-    st_unless_null<3 * V>(out.v_t, (r * n + c) * 3, acc_vt);
+    st_unless_null<3 * V>(out.v, (r * n + c) * 3, plus(acc_v, ld_vecs<V>(add.v, (r * n + c) * 3)));
+    st_unless_null<3 * V>(out.v_t, (r * n + c) * 3, plus(acc_vt, ld_vecs<V>(add.v_t, (r * n + c) * 3)));
 }
 
 // ------------------------------------------------------------------------------------------------ the update
@@ -623,8 +635,9 @@ template <bool DUAL>
 __global__ void __launch_bounds__(256) update_post_fwd_kernel(const float* __restrict__ lrv, const float* __restrict__ ip,
                                                               const float* __restrict__ y, const GroupStats* __restrict__ stats,
                                                               const float* __restrict__ gamma, const float* __restrict__ beta,
-                                                              long R, int N, int n, int groups, float* __restrict__ out_a,
-                                                              float* __restrict__ out_v) {
+                                                              long R, int N, int n, int groups, mg_painn_rows res,
+                                                              float* __restrict__ out_a, float* __restrict__ out_at,
+                                                              float* __restrict__ out_v, float* __restrict__ out_vt) {
     const int quads = n >> 2, cpg = n / groups;
     const long t = (long)blockIdx.x * 256 + threadIdx.x;
     const long r = t / quads;
@@ -658,11 +671,11 @@ __global__ void __launch_bounds__(256) update_post_fwd_kernel(const float* __res
             ovt.set(j, q * wt + (-q * q * q * dot(w, wt)) * w);
         }
     }
-    st4(out_a + r * n + c, oa);
-    st12(out_v + (r * n + c) * 3, ov);
+    st4(out_a + r * n + c, plus(oa, ld_chans<4>(res.a, r * n + c)));
+    st12(out_v + (r * n + c) * 3, plus(ov, ld_vecs<4>(res.v, (r * n + c) * 3)));
     if constexpr (DUAL) {
-        st4(out_a + (R + r) * n + c, oat);
-        st12(out_v + ((R + r) * n + c) * 3, ovt);
+        st4(out_at + r * n + c, plus(oat, ld_chans<4>(res.a_t, r * n + c)));
+        st12(out_vt + (r * n + c) * 3, plus(ovt, ld_vecs<4>(res.v_t, (r * n + c) * 3)));
     }
 }
 
@@ -864,7 +877,7 @@ template <bool DUAL>
 __global__ void __launch_bounds__(256) update_pre_bwd_kernel(const float* __restrict__ lrv, const float* __restrict__ g_ip,
                                                              const float* __restrict__ g_cat, long R, int n, int lanes,
                                                              float* __restrict__ g_lrv, float* __restrict__ g_lrv_max,
-                                                             float* __restrict__ g_xa) {
+                                                             mg_painn_rows add, float* __restrict__ g_xa) {
     const long t = (long)blockIdx.x * 256 + threadIdx.x;
     const long r_raw = t / lanes;
     const bool live = r_raw < R;
@@ -916,8 +929,8 @@ __global__ void __launch_bounds__(256) update_pre_bwd_kernel(const float* __rest
                     st4(g_lrv + (rt * 3 + k) * 3 * n + n + c, grt[k]);
                 }
             }
-            st4(g_xa + r * n + c, ld4(g_cat + r * 2 * n + c));
-            if constexpr (DUAL) st4(g_xa + rt * n + c, ld4(g_cat + rt * 2 * n + c));
+            st4(g_xa + r * n + c, plus(ld4(g_cat + r * 2 * n + c), ld_chans<4>(add.a, r * n + c)));
+            if constexpr (DUAL) st4(g_xa + rt * n + c, plus(ld4(g_cat + rt * 2 * n + c), ld_chans<4>(add.a_t, r * n + c)));
         }
     }
 #pragma unroll
@@ -996,6 +1009,9 @@ static bool combine_aligned(const mg_painn_combine_dual* a) {
     return true;
 }
 
+static mg_painn_rows rows_or_none(const mg_painn_rows* p) { return p ? *p : mg_painn_rows{nullptr, nullptr, nullptr, nullptr}; }
+static bool rows_aligned(const mg_painn_rows& p) { return aligned16(p.a) && aligned16(p.a_t) && aligned16(p.v) && aligned16(p.v_t); }
+
 // Channels of a lane of the message kernels: two, so that a row of 128 channels is a whole wave and a lane's operands leave room for
 // several waves on a SIMD (the adjoint: 153 registers, three waves; with four channels 266, one); four where two would spread a row
 // over two waves (n = 256).  78 000 edges of 4096 nodes in no order, before (four channels a lane) -> now: n = 128 forward
@@ -1005,30 +1021,44 @@ static int combine_channels(int n) { return n <= 128 ? 2 : 4; }
 
 int mg_painn_combine_dual_fwd(const mg_painn_combine_dual* a, const int* node, const int* row_ptr, long n_out, float* out_v,
                               float* out_v_t, float* out_a, float* out_a_t, mg_stream_t stream) {
+    return mg_painn_combine_dual_add_fwd(a, node, row_ptr, n_out, nullptr, out_v, out_v_t, out_a, out_a_t, stream);
+}
+
+int mg_painn_combine_dual_add_fwd(const mg_painn_combine_dual* a, const int* node, const int* row_ptr, long n_out,
+                                  const mg_painn_rows* residual, float* out_v, float* out_v_t, float* out_a, float* out_a_t,
+                                  mg_stream_t stream) {
+    const mg_painn_rows res = rows_or_none(residual);
     MG_REQUIRE(a != nullptr && a->E >= 0 && a->n_rows >= 0 && n_out >= 0 && mg_painn_combine_supported(a->n),
                "mg_painn_combine_dual_fwd: n must be a power of two in 4..256");
     if (n_out == 0) return MG_OK;
     MG_REQUIRE(row_ptr && out_v && out_v_t && out_a && out_a_t && aligned16(out_v) && aligned16(out_v_t) && aligned16(out_a) &&
-                   aligned16(out_a_t) && combine_aligned(a) &&
+                   aligned16(out_a_t) && combine_aligned(a) && rows_aligned(res) &&
                    (a->E == 0 || (a->dist && a->actv && a->v && a->dir && node && a->n_rows > 0)),
                "mg_painn_combine_dual_fwd: null or unaligned pointer");
     const CombineIn in{a->dist, a->dist_t, a->actv, a->actv_t, a->v, a->v_t, a->dir, a->dir_t};
     const int per_lane = combine_channels(a->n);
     hipLaunchKernelGGL(per_lane == 2 ? combine_dual_fwd_kernel<2> : combine_dual_fwd_kernel<4>,
                        dim3((unsigned)(8 * ceil_div(n_out * (a->n / per_lane), 8 * 256))), dim3(256), 0, (hipStream_t)stream, in, node,
-                       a->n_rows, row_ptr, n_out, a->E, a->n, out_v, out_v_t, out_a, out_a_t);
+                       a->n_rows, row_ptr, n_out, a->E, a->n, res, out_v, out_v_t, out_a, out_a_t);
     return check_launch("mg_painn_combine_dual_fwd");
 }
 
 int mg_painn_combine_dual_bwd(const mg_painn_combine_dual* a, const int* row_ptr, const int* order, const float* g_v,
                               const float* g_v_t, const float* g_a, const float* g_a_t, const int* grad_row, long n_grad_rows,
                               const mg_painn_combine_dual_grad* d, mg_stream_t stream) {
+    return mg_painn_combine_dual_add_bwd(a, row_ptr, order, g_v, g_v_t, g_a, g_a_t, grad_row, n_grad_rows, nullptr, d, stream);
+}
+
+int mg_painn_combine_dual_add_bwd(const mg_painn_combine_dual* a, const int* row_ptr, const int* order, const float* g_v,
+                                  const float* g_v_t, const float* g_a, const float* g_a_t, const int* grad_row, long n_grad_rows,
+                                  const mg_painn_rows* added, const mg_painn_combine_dual_grad* d, mg_stream_t stream) {
+    const mg_painn_rows add = rows_or_none(added);
     MG_REQUIRE(a != nullptr && d != nullptr && a->E >= 0 && a->E < (1L << 31) && a->n_rows >= 0 && mg_painn_combine_supported(a->n),
                "mg_painn_combine_dual_bwd: n must be a power of two in 4..256");
     if (a->n_rows == 0) return MG_OK;
     MG_REQUIRE(a->actv && a->v && row_ptr && combine_aligned(a) &&
                    (a->E == 0 || (a->dist && a->dir && g_v && g_v_t && g_a && g_a_t && grad_row && n_grad_rows > 0)) &&
-                   aligned16(g_v) && aligned16(g_v_t) && aligned16(g_a) && aligned16(g_a_t),
+                   aligned16(g_v) && aligned16(g_v_t) && aligned16(g_a) && aligned16(g_a_t) && rows_aligned(add),
                "mg_painn_combine_dual_bwd: null or unaligned pointer");
     for (const float* p : {d->dist, d->dist_t, d->actv, d->actv_t, d->v, d->v_t})
         MG_REQUIRE(aligned16(p), "mg_painn_combine_dual_bwd: gradients must be 16-byte aligned");
@@ -1037,7 +1067,7 @@ int mg_painn_combine_dual_bwd(const mg_painn_combine_dual* a, const int* row_ptr
     const int per_lane = combine_channels(a->n);
     hipLaunchKernelGGL(per_lane == 2 ? combine_dual_bwd_kernel<2> : combine_dual_bwd_kernel<4>,
                        dim3((unsigned)(8 * ceil_div(a->n_rows * (a->n / per_lane), 8 * 256))), dim3(256), 0, (hipStream_t)stream, in, row_ptr, order, a->n_rows, g_v, g_v_t, g_a, g_a_t, grad_row, n_grad_rows, a->E, a->n,
-                       out);
+                       out, add);
     return check_launch("mg_painn_combine_dual_bwd");
 }
 
@@ -1066,12 +1096,24 @@ int mg_painn_update_scratch_floats(int batch, int nodes, int n, int groups, long
 int mg_painn_update_post_fwd(const float* lrv, const float* ip, const float* y, const float* gamma, const float* beta, int batch,
                              int nodes, int n, int groups, float eps, int dual, float* scratch, float* stats, float* out_a,
                              float* out_v, mg_stream_t stream) {
+    const long values = (long)batch * nodes * n;
+    return mg_painn_update_post_add_fwd(lrv, ip, y, gamma, beta, batch, nodes, n, groups, eps, dual, scratch, stats, nullptr, out_a,
+                                        dual && out_a ? out_a + values : nullptr, out_v, dual && out_v ? out_v + 3 * values : nullptr,
+                                        stream);
+}
+
+int mg_painn_update_post_add_fwd(const float* lrv, const float* ip, const float* y, const float* gamma, const float* beta, int batch,
+                                 int nodes, int n, int groups, float eps, int dual, float* scratch, float* stats,
+                                 const mg_painn_rows* residual, float* out_a, float* out_a_t, float* out_v, float* out_v_t,
+                                 mg_stream_t stream) {
+    const mg_painn_rows res = rows_or_none(residual);
     const long R = (long)batch * nodes;
     MG_REQUIRE(batch >= 0 && nodes >= 0 && groups >= 1 && rows_ok(R, n) && n % groups == 0,
                "mg_painn_update_post_fwd: bad shape");
     if (R == 0) return MG_OK;
     MG_REQUIRE(lrv && ip && y && gamma && beta && scratch && stats && out_a && out_v && aligned16(lrv) && aligned16(ip) &&
-                   aligned16(y) && aligned16(out_a) && aligned16(out_v) && aligned16(stats),
+                   aligned16(y) && aligned16(out_a) && aligned16(out_v) && aligned16(stats) && rows_aligned(res) &&
+                   (!dual || (out_a_t && out_v_t && aligned16(out_a_t) && aligned16(out_v_t))),
                "mg_painn_update_post_fwd: null or unaligned pointer");
     const int pieces = (int)ceil_div((long)nodes * (n / groups), kPiece);
     MG_REQUIRE((long)pieces * groups * batch <= 0x7fffffffL, "mg_painn_update_post_fwd: too many boxes");
@@ -1079,7 +1121,7 @@ int mg_painn_update_post_fwd(const float* lrv, const float* ip, const float* y, 
     MG_DUAL_LAUNCH(gn_pieces_kernel, dim3((unsigned)(pieces * groups * batch)), dim3(256), ip, y, R, nodes, n, groups, pieces, scratch);
     hipLaunchKernelGGL(gn_finish_kernel, dim3((unsigned)(batch * groups)), dim3(64), 0, (hipStream_t)stream, scratch, pieces, eps, st);
     MG_DUAL_LAUNCH(update_post_fwd_kernel, dim3((unsigned)ceil_div(R * (n / 4), 256)), dim3(256), lrv, ip, y, st, gamma, beta, R,
-                   nodes, n, groups, out_a, out_v);
+                   nodes, n, groups, res, out_a, out_a_t, out_v, out_v_t);
     return check_launch("mg_painn_update_post_fwd");
 }
 
@@ -1114,14 +1156,20 @@ int mg_painn_update_post_bwd(const float* lrv, const float* ip, const float* y, 
 
 int mg_painn_update_pre_bwd(const float* lrv, const float* g_ip, const float* g_cat, long rows, int n, int dual, float* g_lrv,
                             float* g_lrv_rowmax, float* g_xa, mg_stream_t stream) {
+    return mg_painn_update_pre_add_bwd(lrv, g_ip, g_cat, rows, n, dual, g_lrv, g_lrv_rowmax, nullptr, g_xa, stream);
+}
+
+int mg_painn_update_pre_add_bwd(const float* lrv, const float* g_ip, const float* g_cat, long rows, int n, int dual, float* g_lrv,
+                                float* g_lrv_rowmax, const mg_painn_rows* added, float* g_xa, mg_stream_t stream) {
+    const mg_painn_rows add = rows_or_none(added);
     MG_REQUIRE(rows_ok(rows, n), "mg_painn_update_pre_bwd: n % 4 == 0 expected");
     if (rows == 0) return MG_OK;
     MG_REQUIRE(lrv && g_ip && g_cat && g_lrv && g_lrv_rowmax && g_xa && aligned16(lrv) && aligned16(g_ip) && aligned16(g_cat) &&
-                   aligned16(g_lrv) && aligned16(g_xa),
+                   aligned16(g_lrv) && aligned16(g_xa) && rows_aligned(add),
                "mg_painn_update_pre_bwd: null or unaligned pointer");
     const int lanes = row_lanes(n);
     MG_DUAL_LAUNCH(update_pre_bwd_kernel, dim3(row_blocks(rows, lanes)), dim3(256), lrv, g_ip, g_cat, rows, n, lanes, g_lrv,
-                   g_lrv_rowmax, g_xa);
+                   g_lrv_rowmax, add, g_xa);
     return check_launch("mg_painn_update_pre_bwd");
 }
 

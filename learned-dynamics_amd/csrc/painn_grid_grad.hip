@@ -134,7 +134,7 @@ __global__ void __launch_bounds__(1024) grid_node_grad_kernel(
     const int* __restrict__ row_ptr, const int* __restrict__ from, const int* __restrict__ node_order, long n_nodes, long E,
     const float4* __restrict__ rec, const float* __restrict__ table, int tab_rows, const float* __restrict__ g_v,
     const float* __restrict__ g_a, const float* __restrict__ actv, const float* __restrict__ v, int n,
-    float* __restrict__ d_actv, float* __restrict__ d_v) {
+    const float* __restrict__ add_v, float* __restrict__ d_actv, float* __restrict__ d_v) {
     extern __shared__ float tab[];                            // (tab_rows + 3) x kSliceRowF
     const int n_slices = n / kSliceChan;
     const int slice = blockIdx.x % n_slices;
@@ -207,7 +207,11 @@ __global__ void __launch_bounds__(1024) grid_node_grad_kernel(
         float s0 = vq * sA, s1 = vq * sB;                     // v . M0, v . M1: over the lanes q = 0..2 of the channel
         s0 += __shfl_xor(s0, 4); s1 += __shfl_xor(s1, 4);
         s0 += __shfl_xor(s0, 8); s1 += __shfl_xor(s1, 8);
-        if (d_v && q < 3) d_v[(node * n + ch) * 3 + q] = a0 * sA + a1 * sB;
+        if (d_v && q < 3) {
+            const long at = (node * n + ch) * 3 + q;
+            const float own = a0 * sA + a1 * sB;
+            d_v[at] = add_v ? own + add_v[at] : own;
+        }
         if (d_actv) {
             if (q == 3) { d_actv[row4 + 2 * n] = sA; d_actv[row4 + 3 * n] = sB; }
             else if (q < 2) d_actv[row4 + q * n] = q ? s1 : s0;
@@ -474,6 +478,14 @@ int mg_painn_grid_node_grad(const int* row_ptr, const int* order, const int* src
                             const float* r_ij, const float* table, int table_rows, float period, float epsilon, const float* g_v,
                             const float* g_a, const float* actv, const float* v, int n, void* workspace, float* d_actv, float* d_v,
                             mg_stream_t stream) {
+    return mg_painn_grid_node_add_grad(row_ptr, order, src, node_order, n_nodes, n_edges, r_ij, table, table_rows, period, epsilon, g_v,
+                                       g_a, actv, v, n, workspace, nullptr, d_actv, d_v, stream);
+}
+
+int mg_painn_grid_node_add_grad(const int* row_ptr, const int* order, const int* src, const int* node_order, int n_nodes, long n_edges,
+                                const float* r_ij, const float* table, int table_rows, float period, float epsilon, const float* g_v,
+                                const float* g_a, const float* actv, const float* v, int n, void* workspace, const float* add_v,
+                                float* d_actv, float* d_v, mg_stream_t stream) {
     MG_REQUIRE(n_nodes >= 0 && n_edges >= 0 && n_edges < (1L << 31) && period > 0.f && mg_painn_grid_grad_supported(table_rows, n),
                "mg_painn_grid_node_grad: bad argument");
     if (n_nodes == 0) return MG_OK;
@@ -494,7 +506,7 @@ int mg_painn_grid_node_grad(const int* row_ptr, const int* order, const int* src
     if (groups > max_groups) groups = max_groups;
     hipLaunchKernelGGL(grid_node_grad_kernel, dim3((unsigned)(groups * n_slices)), dim3(1024),
                        (size_t)(table_rows + kSliceExtraRows) * kSliceRowF * sizeof(float), st, row_ptr, from, node_order,
-                       (long)n_nodes, n_edges, rec, table, table_rows, g_v, g_a, actv, v, n, d_actv, d_v);
+                       (long)n_nodes, n_edges, rec, table, table_rows, g_v, g_a, actv, v, n, add_v, d_actv, d_v);
     return check_launch("mg_painn_grid_node_grad");
 }
 

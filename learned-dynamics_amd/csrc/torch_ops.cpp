@@ -1292,22 +1292,37 @@ mg_painn_combine_dual combine_in(const std::vector<OptTensor>& in) {
     return {fp(in[0]), fp(in[1]), fp(in[2]), fp(in[3]), fp(in[4]), fp(in[5]), fp(in[6]), fp(in[7]), E, rows, (int)n};
 }
 
-Tensors combine_dual_fwd(const std::vector<OptTensor>& in, const at::Tensor& node, const at::Tensor& row_ptr, int64_t n_out) {
+// The rows a, a_t, v, v_t (any may be missing) that a layer adds to its results
+mg_painn_rows rows_in(const std::vector<OptTensor>& in, int64_t rows, int64_t n) {
+    TORCH_CHECK(in.size() == 4, "four arrays of rows expected");
+    for (int k = 0; k < 4; k++) {
+        if (!in[k].has_value()) continue;
+        check_input(*in[k], "rows to add");
+        TORCH_CHECK(in[k]->numel() == rows * n * (k < 2 ? 1 : 3), "rows to add: wrong shape");
+    }
+    return {fp(in[0]), fp(in[1]), fp(in[2]), fp(in[3])};
+}
+
+// residual: nothing, or a, a_t, v, v_t.  Each result on storage of its own: a dual tensor copies a tangent that shares its value's.
+Tensors combine_dual_fwd(const std::vector<OptTensor>& in, const at::Tensor& node, const at::Tensor& row_ptr, int64_t n_out,
+                         const std::vector<OptTensor>& residual) {
     const mg_painn_combine_dual a = combine_in(in);
     check_input(node, "node", at::kInt);
     check_input(row_ptr, "row_ptr", at::kInt);
     TORCH_CHECK(node.numel() == a.E && row_ptr.numel() == n_out + 1, "combine_dual: index sizes");
     const at::Tensor& like = *in[0];
     c10::hip::HIPGuardMasqueradingAsCUDA guard(like.device());
-    at::Tensor v = floats(like, {2 * n_out, a.n, 3}), s = floats(like, {2 * n_out, a.n});
-    check(mg_painn_combine_dual_fwd(&a, node.data_ptr<int>(), row_ptr.data_ptr<int>(), n_out, fp(v), fp(v) + n_out * a.n * 3, fp(s),
-                                    fp(s) + n_out * a.n, stream_of(like)));
-    const std::vector<int64_t> sv{n_out, a.n, 3}, sa{n_out, a.n};
-    return {on_storage(v, 0, sv), on_storage(s, 0, sa), *second_half(v, sv, true), *second_half(s, sa, true)};
+    mg_painn_rows res{};
+    if (!residual.empty()) res = rows_in(residual, n_out, a.n);
+    Tensors out{floats(like, {n_out, a.n, 3}), floats(like, {n_out, a.n}), floats(like, {n_out, a.n, 3}), floats(like, {n_out, a.n})};
+    check(mg_painn_combine_dual_add_fwd(&a, node.data_ptr<int>(), row_ptr.data_ptr<int>(), n_out, &res, fp(out[0]), fp(out[2]),
+                                        fp(out[1]), fp(out[3]), stream_of(like)));
+    return out;
 }
 
 std::vector<OptTensor> combine_dual_bwd(const std::vector<OptTensor>& in, const at::Tensor& row_ptr, const OptTensor& order,
-                                        const Tensors& g, const at::Tensor& grad_row, int64_t n_grad_rows, const std::vector<bool>& want) {
+                                        const Tensors& g, const at::Tensor& grad_row, int64_t n_grad_rows, const std::vector<bool>& want,
+                                        bool residual) {
     const mg_painn_combine_dual a = combine_in(in);
     check_input(row_ptr, "row_ptr", at::kInt);
     check_input(grad_row, "grad_row", at::kInt);
@@ -1337,8 +1352,12 @@ std::vector<OptTensor> combine_dual_bwd(const std::vector<OptTensor>& in, const 
         p[k + 1] = second ? fp(buf) + in[k]->numel() : nullptr;
     }
     const mg_painn_combine_dual_grad d{p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7]};
-    check(mg_painn_combine_dual_bwd(&a, row_ptr.data_ptr<int>(), order.has_value() ? order->data_ptr<int>() : nullptr, fp(g[0]),
-                                    fp(g[2]), fp(g[1]), fp(g[3]), grad_row.data_ptr<int>(), n_grad_rows, &d, stream_of(like)));
+    // (v went past the message as well: its gradient is the sum's own plus that of the result it was added to)
+    TORCH_CHECK(!residual || n_grad_rows == a.n_rows, "combine_dual: rows to add");
+    const mg_painn_rows add{nullptr, nullptr, residual ? fp(g[0]) : nullptr, residual ? fp(g[2]) : nullptr};
+    check(mg_painn_combine_dual_add_bwd(&a, row_ptr.data_ptr<int>(), order.has_value() ? order->data_ptr<int>() : nullptr, fp(g[0]),
+                                        fp(g[2]), fp(g[1]), fp(g[3]), grad_row.data_ptr<int>(), n_grad_rows, &add, &d,
+                                        stream_of(like)));
     return out;
 }
 
@@ -1360,7 +1379,7 @@ std::pair<at::Tensor, at::Tensor> vector_rows(const at::Tensor& x_v, const OptTe
 std::tuple<Tensors, std::vector<OptTensor>> painn_update_train_fwd(const at::Tensor& x_a, const OptTensor& x_at, const at::Tensor& x_v,
                                                                    const OptTensor& x_vt, const Tensors& lrv_W, const Tensors& W,
                                                                    const Tensors& b, int groups, const at::Tensor& gamma,
-                                                                   const at::Tensor& beta, double eps) {
+                                                                   const at::Tensor& beta, double eps, bool residual) {
     check_input(x_a, "x_a");
     check_input(x_v, "x_v");
     check_input(gamma, "gamma");
@@ -1384,14 +1403,16 @@ std::tuple<Tensors, std::vector<OptTensor>> painn_update_train_fwd(const at::Ten
     long fwd = 0, bwd = 0;
     check(mg_painn_update_scratch_floats((int)B, (int)N, (int)n, groups, &fwd, &bwd));
     at::Tensor scratch = floats(x_a, {std::max<int64_t>(fwd, 1)}), stats = floats(x_a, {B * groups, 4});
-    at::Tensor out_a = floats(x_a, {copies * R, n}), out_v = floats(x_a, {copies * R, n, 3});
-    check(mg_painn_update_post_fwd(fp(lrv), fp(ip), fp(y), fp(gamma), fp(beta), (int)B, (int)N, (int)n, groups, (float)eps, dual,
-                                   fp(scratch), fp(stats), fp(out_a), fp(out_v), st));
-    Tensors out{on_storage(out_a, 0, x_a.sizes()), on_storage(out_v, 0, x_v.sizes())};
-    if (dual) {
-        out.push_back(*second_half(out_a, x_a.sizes(), true));
-        out.push_back(*second_half(out_v, x_v.sizes(), true));
+    Tensors out;                                 // (each on storage of its own, as combine_dual_fwd's)
+    for (int k = 0; k < copies; k++) {
+        out.push_back(floats(x_a, x_a.sizes()));
+        out.push_back(floats(x_v, x_v.sizes()));
     }
+    mg_painn_rows res{};
+    if (residual) res = rows_in({OptTensor(x_a), x_at, OptTensor(x_v), x_vt}, R, n);
+    check(mg_painn_update_post_add_fwd(fp(lrv), fp(ip), fp(y), fp(gamma), fp(beta), (int)B, (int)N, (int)n, groups, (float)eps, dual,
+                                       fp(scratch), fp(stats), &res, fp(out[0]), dual ? fp(out[2]) : nullptr, fp(out[1]),
+                                       dual ? fp(out[3]) : nullptr, st));
     std::vector<OptTensor> saved{OptTensor(W_lrv), OptTensor(x2), OptTensor(x2max), OptTensor(lrv), OptTensor(ip), OptTensor(cat),
                                  OptTensor(y), OptTensor(stats), lrv_planes[1]};
     saved.insert(saved.end(), mlp_saved.begin(), mlp_saved.end());
@@ -1401,7 +1422,8 @@ std::tuple<Tensors, std::vector<OptTensor>> painn_update_train_fwd(const at::Ten
 // gradients of x_a, x_v and their tangents, of l, r, v, of gamma and beta, and of the MLP's weights and biases
 std::tuple<std::vector<OptTensor>, Tensors> painn_update_train_bwd(const at::Tensor& g_a, const OptTensor& g_at, const at::Tensor& g_v,
                                                                    const OptTensor& g_vt, const Tensors& W, int groups,
-                                                                   const at::Tensor& gamma, const std::vector<OptTensor>& saved) {
+                                                                   const at::Tensor& gamma, const std::vector<OptTensor>& saved,
+                                                                   bool residual) {
     const bool dual = g_at.has_value();
     check_input(g_a, "gradient of out_a");
     check_input(g_v, "gradient of out_v");
@@ -1424,7 +1446,9 @@ std::tuple<std::vector<OptTensor>, Tensors> painn_update_train_bwd(const at::Ten
                                    fp(d_beta), st));
     auto [g_cat, mlp_params] = mlp_rows_bwd(g_y, OptTensor(g_y_max), cat, R, W, mlp_saved, true, true);
     at::Tensor g_xa = floats(g_a, {copies * R, n});
-    check(mg_painn_update_pre_bwd(fp(lrv), fp(g_ip), fp(*g_cat), R, (int)n, dual, fp(g_lrv), fp(g_lrv_max), fp(g_xa), st));
+    mg_painn_rows add{};
+    if (residual) add = rows_in({OptTensor(g_a), g_at, OptTensor(g_v), g_vt}, R, n);
+    check(mg_painn_update_pre_add_bwd(fp(lrv), fp(g_ip), fp(*g_cat), R, (int)n, dual, fp(g_lrv), fp(g_lrv_max), &add, fp(g_xa), st));
     const OptTensor g_bound(g_lrv_max);
     const at::Tensor dW = rows_wgrad(g_lrv, x2, 0, false, g_bound, saved[2]).first;
     at::Tensor g_xv;
@@ -1439,6 +1463,10 @@ std::tuple<std::vector<OptTensor>, Tensors> painn_update_train_bwd(const at::Ten
     const std::vector<int64_t> sv{B, N, n, 3};
     std::vector<OptTensor> g_x{OptTensor(on_storage(g_xa, 0, g_a.sizes())), second_half(g_xa, g_a.sizes(), dual),
                                OptTensor(on_storage(g_xv, 0, sv)), second_half(g_xv, sv, dual)};
+    if (residual) {
+        g_x[2]->add_(g_v.view(sv));
+        if (dual) g_x[3]->add_(g_vt->view(sv));
+    }
     Tensors params{on_storage(dW, 0, {n, n}), on_storage(dW, n * n, {n, n}), on_storage(dW, 2 * n * n, {n, n}), d_gamma, d_beta};
     params.insert(params.end(), mlp_params.begin(), mlp_params.end());
     return {g_x, params};
@@ -1468,7 +1496,7 @@ std::tuple<OptTensor, OptTensor, OptTensor> painn_grid_message_bwd(const at::Ten
                                                                    const at::Tensor& row_ptr, const OptTensor& order,
                                                                    const OptTensor& node_order, double period, double epsilon,
                                                                    bool want_table, bool want_actv, bool want_v,
-                                                                   const OptTensor& src_row_ptr) {
+                                                                   const OptTensor& src_row_ptr, bool residual) {
     for (const at::Tensor& t : {table, actv, actv_sliced, v, r_ij, g_v, g_a}) check_input(t, "operand of the message");
     for (const at::Tensor& t : {src, dst, row_ptr}) check_input(t, "index", at::kInt);
     for (const OptTensor& t : {order, node_order, src_row_ptr})
@@ -1489,9 +1517,10 @@ std::tuple<OptTensor, OptTensor, OptTensor> painn_grid_message_bwd(const at::Ten
     if (want_actv || want_v) {
         if (want_actv) d_actv = floats(v, {N, 4 * n});
         if (want_v) d_v = floats(v, v.sizes());
-        check(mg_painn_grid_node_grad(row_ptr.data_ptr<int>(), ints(order), src.data_ptr<int>(), ints(node_order), (int)N, E, fp(r_ij),
-                                      fp(table), (int)rows, (float)period, (float)epsilon, fp(g_v), fp(g_a), fp(actv), fp(v), (int)n,
-                                      ws.data_ptr(), want_actv ? fp(*d_actv) : nullptr, want_v ? fp(*d_v) : nullptr, st));
+        // (v went past the message as well)
+        check(mg_painn_grid_node_add_grad(row_ptr.data_ptr<int>(), ints(order), src.data_ptr<int>(), ints(node_order), (int)N, E,
+                                      fp(r_ij), fp(table), (int)rows, (float)period, (float)epsilon, fp(g_v), fp(g_a), fp(actv), fp(v),
+                                      (int)n, ws.data_ptr(), residual ? fp(g_v) : nullptr, want_actv ? fp(*d_actv) : nullptr, want_v ? fp(*d_v) : nullptr, st));
     }
     if (want_table) {
         d_table = floats(v, table.sizes());

@@ -302,6 +302,16 @@ def mlp_silu(mlp, x):
     return out if t is None else fwAD.make_dual(*out)
 
 
+def _mlp_silu_pair(mlp, x):
+    """mlp_silu's (value, tangent or None) for a caller that takes them apart: a dual tensor would copy the tangent."""
+    params = _mlp_parameters(mlp)
+    p, t = (_dense(z) for z in _unpack(x))
+    if not (_fused(params, p, t) and p.shape[-1] % 4 == 0):
+        return _unpack(_mlp_rows(params, x))
+    out = _MlpSilu.apply(p, t, None, *params)
+    return (out, None) if t is None else out
+
+
 class _MlpLeaky(torch.autograd.Function):
     """bee_layers.MLP on rows: the layers as one kernel each way, the direct map added to their result.  params: weight and bias of
     the three layers, then the direct map's weight."""
@@ -571,32 +581,39 @@ class _PainnCombineGrad(torch.autograd.Function):
 class _PainnCombineDual(torch.autograd.Function):
     """_PainnCombine of values and tangents at once: (dist, dist_t, actv, actv_t, v, v_t, direction, direction_t) -> (out_v,
     out_a, out_v_t, out_a_t), any tangent None.  One kernel each way, where the rule of _PainnCombine.jvp makes one call
-    for the values and one for each argument with a tangent, and as many in the backward pass."""
+    for the values and one for each argument with a tangent, and as many in the backward pass.
+    x, x_t: None, or the rows that out_a and its tangent are added to; v and v_t are then added to out_v and its tangent, and the
+    adjoint's kernel adds both gradients of v."""
 
     @staticmethod
-    def forward(ctx, by_dst, by_src, *args):
-        ctx.by_dst, ctx.by_src = by_dst, by_src
+    def forward(ctx, by_dst, by_src, x, x_t, *args):
+        ctx.by_dst, ctx.by_src, ctx.residual = by_dst, by_src, x is not None
         ctx.save_for_backward(*args)
-        return ops.painn_combine_dual_fwd(args, by_dst.index, by_src.row_ptr, by_src.n_rows)
+        return ops.painn_combine_dual_fwd(args, by_dst.index, by_src.row_ptr, by_src.n_rows,
+                                          (x, x_t, args[4], args[5]) if ctx.residual else ())
 
     @staticmethod
     def backward(ctx, *grads):
-        args, need = ctx.saved_tensors, ctx.needs_input_grad[2:]
+        args, need, residual = ctx.saved_tensors, ctx.needs_input_grad[4:], ctx.residual
         by_dst, by_src = ctx.by_dst, ctx.by_src
+        past = tuple(g if nd else None for g, nd in zip((grads[1], grads[3]), ctx.needs_input_grad[2:4]))
         if torch.is_grad_enabled():
-            return (None, None) + _recorded_gradients(lambda *a: _combine_pairs(a, by_dst, by_src), args, need, grads)
+            return (None, None, *past) + _recorded_gradients(lambda *a: _combine_pairs(a, by_dst, by_src, residual), args, need, grads)
         outs = ops.painn_combine_dual_bwd(args, by_dst.row_ptr, by_dst.perm, [g.contiguous() for g in grads], by_src.index,
-                                          by_src.n_rows, need)
-        return (None, None) + tuple(o if nd else None for o, nd in zip(outs, need))
+                                          by_src.n_rows, need, residual)
+        return (None, None, *past) + tuple(o if nd else None for o, nd in zip(outs, need))
 
 
-def _combine_pairs(args, by_dst, by_src):
-    """_PainnCombineDual out of calls of _PainnCombine."""
+def _combine_pairs(args, by_dst, by_src, residual=False):
+    """_PainnCombineDual out of calls of _PainnCombine (of the rows that results are added to, v and v_t alone)."""
     values, tangents = args[0::2], args[1::2]
     out_v, out_a = _PainnCombine.apply(*values, by_dst, by_src, _TERMS_ALL)
     pairs = [_PainnCombine.apply(*(t if j == k else v for j, v in enumerate(values)), by_dst, by_src, terms)
              for k, (t, terms) in enumerate(zip(tangents, (_TERMS_ALL, _TERMS_ALL, _TERMS_V, _TERMS_DIR))) if t is not None]
-    return out_v, out_a, _sum_opt([p[0] for p in pairs]), _sum_opt([p[1] for p in pairs])
+    out_vt, out_at = _sum_opt([p[0] for p in pairs]), _sum_opt([p[1] for p in pairs])
+    if residual:
+        out_v, out_vt = args[4] + out_v, out_vt if args[5] is None else args[5] + out_vt
+    return out_v, out_a, out_vt, out_at
 
 
 def painn_combine(graph, dist, actv_node, v_node, direction):
@@ -767,10 +784,10 @@ class _EdgeEncode(torch.autograd.Function):
         return g_r if need[0] else None, g_rt if need[1] else None, None, None, None
 
 
-def _message_edges(msg, graph, actv, x_v, r_ij):
-    """The message with the filter MLP on every edge, or None where the fused functions do not take it."""
+def _message_edges(msg, graph, actv, x_v, r_ij, x_a=None):
+    """The message with the filter MLP on every edge, or None where the fused functions do not take it.  actv: value and tangent."""
     params, n = _mlp_parameters(msg.mlp_dist), msg.n
-    (r, r_t), (a, a_t), (v, v_t) = _unpack(r_ij), _unpack(actv), _unpack(x_v)
+    (r, r_t), (a, a_t), (v, v_t) = _unpack(r_ij), actv, _unpack(x_v)
     r, r_t = r.contiguous(), _dense(r_t)
     flat = [_dense(t if t is None else gl._flat_nodes(graph, t)) for t in (a, a_t, v, v_t)]
     if not (ops.painn_combine_supported(n) and msg.n_rbf % 4 == 0 and _fused(params, r, r_t, *flat)):
@@ -781,20 +798,28 @@ def _message_edges(msg, graph, actv, x_v, r_ij):
     else:
         enc, enc_t, direction, direction_t, bound = _EdgeEncode.apply(r, r_t, msg.n_rbf, msg.r0, msg.epsilon)
         dist, dist_t = _MlpSilu.apply(enc, enc_t, bound, *params)
-    return _combine_flat(graph, dist, dist_t, *flat, direction, direction_t)
+    return _combine_flat(graph, dist, dist_t, *flat, direction, direction_t, x_a, x_v)
 
 
-def _combine_flat(graph, dist, dist_t, a, a_t, v, v_t, direction, direction_t):
-    """(out_a, out_v), with tangents where an operand has one, from operands per edge and per flat node."""
+def _combine_flat(graph, dist, dist_t, a, a_t, v, v_t, direction, direction_t, x_a=None, x_v=None):
+    """(out_a, out_v), with tangents where an operand has one, from operands per edge and per flat node; added to x_a and x_v (v is
+    x_v by flat nodes) unless x_a is None."""
+    x = x_t = None
     if all(t is None for t in (dist_t, a_t, v_t, direction_t)):
         pairs = [(o, None) for o in _PainnCombine.apply(dist, a, v, direction, graph.by_dst, graph.by_src, _TERMS_ALL)]
     else:
-        o_v, o_a, o_vt, o_at = _PainnCombineDual.apply(graph.by_dst, graph.by_src, dist, dist_t, a, a_t, v, v_t, direction,
+        if x_a is not None:
+            x, x_t = (_dense(t if t is None else gl._flat_nodes(graph, t)) for t in _unpack(x_a))
+            rows = graph.by_src.n_rows
+            if not (v.shape[0] == rows and all(t is None or (t.dtype == v.dtype and t.shape == (rows, v.shape[1]) and t.data_ptr() % 16 == 0)
+                                               for t in (x, x_t))):
+                x = x_t = None
+        o_v, o_a, o_vt, o_at = _PainnCombineDual.apply(graph.by_dst, graph.by_src, x, x_t, dist, dist_t, a, a_t, v, v_t, direction,
                                                        direction_t)
         pairs = [(o_v, o_vt), (o_a, o_at)]
     out_v, out_a = (_dual(*(t if t is None else t.reshape(graph.batch, graph.nodes, *t.shape[1:]) for t in pair))
                     for pair in pairs)
-    return out_a, out_v
+    return (add(x_a, out_a), add(x_v, out_v)) if x_a is not None and x is None else (out_a, out_v)
 
 
 _SLICE_PERMUTATIONS = {}
@@ -815,42 +840,48 @@ class _PainnGridMessage(torch.autograd.Function):
     kernel for the gradients of actv and v and one, over the edges sorted by grid row, for the grid's
     (mg_painn_grid_node_grad, mg_painn_grid_table_grad: nothing per edge is stored); for larger grids the gradient kernel of
     the unfused formulation with the filter of every edge interpolated again inside it (mg_painn_combine_bwd_rows), then
-    the scatter into the grid.  A recorded backward pass differentiates the unfused formulation instead."""
+    the scatter into the grid.  A recorded backward pass differentiates the unfused formulation instead.
+    x (nodes, n): None, or the rows that out_a is added to; v is then added to out_v, and the kernel that writes the gradient of v
+    adds that of out_v."""
 
     @staticmethod
-    def forward(ctx, table, actv, v, r_ij, graph, period, epsilon):
-        ctx.graph, ctx.period, ctx.epsilon = graph, period, epsilon
+    def forward(ctx, table, actv, v, r_ij, x, graph, period, epsilon):
+        ctx.graph, ctx.period, ctx.epsilon, ctx.residual = graph, period, epsilon, x is not None
         table, actv, v = table.contiguous(), actv.contiguous(), v.contiguous()
+        res = () if x is None else (x.contiguous(), v)
         actv_s = None
         n = v.size(1)
         if table.size(0) <= ops.PAINN_SLICED_MAX_ROWS and n % ops.PAINN_SLICE == 0:
             # the grid fits in LDS: the kernel that holds it there takes actv with its columns grouped slice by slice
             actv_s = actv[:, _slice_permutation(n, actv.device)].contiguous()
-            out_a, out_v = ops.painn_table_message_sliced(graph.row_ptr, graph.dst32, r_ij, table, period, actv_s, v, epsilon,
+            out_a, out_v = ops.painn_table_message_sliced(graph.row_ptr, graph.dst32, r_ij, table, period, actv_s, v, epsilon, *res,
                                                           node_order=getattr(graph, "cell_order", None))
         else:
-            out_a, out_v = ops.painn_table_message(graph.row_ptr, graph.dst32, r_ij, table, period, actv, v, epsilon)
+            out_a, out_v = ops.painn_table_message(graph.row_ptr, graph.dst32, r_ij, table, period, actv, v, epsilon, *res)
         ctx.save_for_backward(table, actv, v, r_ij, actv_s if ctx.needs_input_grad[0] else None)
         return out_v, out_a
 
     @staticmethod
     def backward(ctx, g_v, g_a):
         table, actv, v, r_ij, actv_s = ctx.saved_tensors
-        graph, need = ctx.graph, ctx.needs_input_grad
+        graph, need, residual = ctx.graph, ctx.needs_input_grad, ctx.residual
+        past = (None, g_a if need[4] else None, None, None, None)
         if torch.is_grad_enabled():
             with torch.enable_grad():
                 leaves = [t if t.requires_grad else t.detach().requires_grad_() for t in (table, actv, v)]
                 out = _grid_message_unfused(*leaves, r_ij, graph, ctx.period, ctx.epsilon)
+                if residual:
+                    out = (out[0] + leaves[2], out[1])
                 grads = torch.autograd.grad(out, leaves, (g_v, g_a), create_graph=True, allow_unused=True)
-            return tuple(g if nd else None for g, nd in zip(grads, need)) + (None, None, None, None)
+            return tuple(g if nd else None for g, nd in zip(grads, need)) + past
         by_dst, by_src = graph.by_dst, graph.by_src
         if ops.painn_grid_grad_supported(table.size(0), v.size(1)) and all(t.data_ptr() % 16 == 0 for t in (table, v, actv)):
             # (the sliced rows are read for the grid's gradient only)
             grads = ops.painn_grid_message_bwd(table, actv, actv if actv_s is None else actv_s, v, r_ij, g_v.contiguous(),
                                                g_a.contiguous(), graph.src32, graph.dst32, by_dst.row_ptr, by_dst.perm,
                                                getattr(graph, "cell_order", None), ctx.period, ctx.epsilon, need[0], need[1],
-                                               need[2], graph.row_ptr)
-            return (*grads, None, None, None, None)
+                                               need[2], graph.row_ptr, residual)
+            return (*grads, *past)
         d = torch.linalg.vector_norm(r_ij, dim=-1).contiguous()
         want = (bool(need[0]), bool(need[1]), bool(need[2]), False)
         # (actv and v are read at an edge's destination: their gradients are summed over a destination's edges inside)
@@ -864,7 +895,8 @@ class _PainnGridMessage(torch.autograd.Function):
             perm, bucket_ptr = ops.painn_table_sorted_edges(d, rows, ctx.period)
             d_table = ops.painn_table_interp_bwd(d_dist, None, d, ctx.period, perm, bucket_ptr, want_length_grad=False,
                                                  order=0, table_rows=rows)[0]
-        return (d_table, d_actv if need[1] else None, dv if need[2] else None, None, None, None, None)
+        dv = (dv + g_v.reshape(dv.shape) if residual else dv) if need[2] else None
+        return (d_table, d_actv if need[1] else None, dv, *past)
 
 
 def _grid_message_unfused(table, actv, v, r_ij, graph, period, epsilon):
@@ -873,62 +905,69 @@ def _grid_message_unfused(table, actv, v, r_ij, graph, period, epsilon):
                                graph.by_dst, graph.by_src, _TERMS_ALL)
 
 
-def painn_message(msg, graph, x_a, x_v, r_ij):
-    """archs/meanflow_painn8.py:85-100"""
+def painn_message(msg, graph, x_a, x_v, r_ij, residual=False):
+    """archs/meanflow_painn8.py:85-100; (x_a + da, x_v + dv) with residual.  The kernels that sum over a node's edges then add the node's
+    own row, and their adjoints the gradient that goes past the message (a step of three blocks on 4
+    systems of 1024 atoms, 128 channels, values and tangents: 99 launches and 260 us less, with the copies of the tangents)."""
     # the MLP acts on rows, so it commutes with the gather: N rows go through it, not E (the reference gathers first),
     # and the gathers themselves are folded into the combining kernel
-    actv = mlp_silu(msg.mlp_actv, x_a)
+    actv = _mlp_silu_pair(msg.mlp_actv, x_a)
     rows = _filter_grid_rows(msg, r_ij)
     n = x_v.size(-2)
     if (rows and n % 4 == 0 and ops.painn_combine_supported(n) and not any(has_tangent(t) for t in (x_a, x_v))
             and r_ij.is_contiguous() and not getattr(graph, "padded", False)):
         table = mlp_silu(msg.mlp_dist, msg._grid_encoding(rows, 0.0, r_ij.device))
-        out_v, out_a = _PainnGridMessage.apply(table, gl._flat_nodes(graph, actv), gl._flat_nodes(graph, x_v), r_ij, graph,
+        flat_v, flat_a = gl._flat_nodes(graph, x_v), gl._flat_nodes(graph, x_a) if residual else None
+        inside = residual and all(t.data_ptr() % 16 == 0 for t in (flat_a, flat_v))
+        out_v, out_a = _PainnGridMessage.apply(table, gl._flat_nodes(graph, actv[0]), flat_v, r_ij, flat_a if inside else None, graph,
                                                2.0 * msg.r0, msg.epsilon)
-        return (out_a.reshape(graph.batch, graph.nodes, *out_a.shape[1:]),
-                out_v.reshape(graph.batch, graph.nodes, *out_v.shape[1:]))
+        out_a, out_v = (t.reshape(graph.batch, graph.nodes, *t.shape[1:]) for t in (out_a, out_v))
+        return (add(x_a, out_a), add(x_v, out_v)) if residual and not inside else (out_a, out_v)
+    x = x_a if residual else None
     if not rows and not getattr(graph, "padded", False):
-        out = _message_edges(msg, graph, actv, x_v, r_ij)
+        out = _message_edges(msg, graph, actv, x_v, r_ij, x)
         if out is not None:
             return out
     dist, direction = painn_filter(msg, r_ij), _unit_vectors(r_ij, msg.epsilon)
-    if ops.painn_combine_supported(n) and any(has_tangent(t) for t in (actv, x_v)) and not has_tangent(dist):
-        flat = [_dense(t if t is None else gl._flat_nodes(graph, t)) for t in (*_unpack(actv), *_unpack(x_v))]
+    if ops.painn_combine_supported(n) and (actv[1] is not None or has_tangent(x_v)) and not has_tangent(dist):
+        flat = [_dense(t if t is None else gl._flat_nodes(graph, t)) for t in (*actv, *_unpack(x_v))]
         if all(t is None or t.data_ptr() % 16 == 0 for t in (*flat, dist)):
-            return _combine_flat(graph, dist.contiguous(), None, *flat, direction.contiguous(), None)
-    out_v, out_a = painn_combine(graph, dist, actv, x_v, direction)
-    return out_a, out_v
+            return _combine_flat(graph, dist.contiguous(), None, *flat, direction.contiguous(), None, x, x_v)
+    out_v, out_a = painn_combine(graph, dist, _dual(*actv), x_v, direction)
+    return (add(x_a, out_a), add(x_v, out_v)) if residual else (out_a, out_v)
 
 
 class _PainnUpdate(torch.autograd.Function):
-    """painn.Update, values alone or values and tangents: one call into the C++ binding for each direction."""
+    """painn.Update, values alone or values and tangents: one call into the C++ binding for each direction.
+    residual: the results are added to x_a and x_v, and the gradients of these are the sums of both."""
 
     @staticmethod
-    def forward(ctx, upd, x_a, x_at, x_v, x_vt, *params):
-        ctx.upd = upd
+    def forward(ctx, upd, residual, x_a, x_at, x_v, x_vt, *params):
+        ctx.upd, ctx.residual = upd, residual
         outs, rows = ops.painn_update_train_fwd(x_a, x_at, x_v, x_vt, params[:3], params[5::2], params[6::2], upd.gn.groups,
-                                                params[3], params[4], upd.gn.epsilon)
+                                                params[3], params[4], upd.gn.epsilon, residual)
         ctx.save_for_backward(x_a, x_at, x_v, x_vt, *params, *(rows if any(ctx.needs_input_grad) else ()))
         ctx.set_materialize_grads(False)
         return tuple(outs)
 
     @staticmethod
     def backward(ctx, g_a, g_v, g_at=None, g_vt=None):
-        upd, need = ctx.upd, list(ctx.needs_input_grad)
+        upd, residual, need = ctx.upd, ctx.residual, list(ctx.needs_input_grad[1:])
         x_a, x_at, x_v, x_vt, *saved = ctx.saved_tensors
         params, rows = saved[:11], saved[11:]
         if all(g is None for g in (g_a, g_v, g_at, g_vt)):
-            return (None,) * len(need)
+            return (None,) * (1 + len(need))
         if torch.is_grad_enabled():
             def pieces(x_a, x_at, x_v, x_vt, *params):
                 if x_vt is None:
-                    return _update_pieces(upd, params, x_a, x_v)
-                split = lambda: tuple(zip(*(fwAD.unpack_dual(o) for o in _update_pieces(upd, params, _dual(x_a, x_at), _dual(x_v, x_vt)))))
+                    return _update_pieces(upd, params, x_a, x_v, residual=residual)
+                split = lambda: tuple(zip(*(fwAD.unpack_dual(o) for o in _update_pieces(upd, params, _dual(x_a, x_at), _dual(x_v, x_vt),
+                                                                                        residual=residual))))
                 if getattr(fwAD, "_current_level", 0) >= 0:
                     return sum(split(), ())
                 with fwAD.dual_level():
                     return sum(split(), ())
-            return (None,) + _recorded_gradients(pieces, (x_a, x_at, x_v, x_vt, *params), need[1:], (g_a, g_v, g_at, g_vt))
+            return (None, None) + _recorded_gradients(pieces, (x_a, x_at, x_v, x_vt, *params), need[1:], (g_a, g_v, g_at, g_vt))
         # (a result that nothing depends on leaves what only it depends on without a gradient, as separate functions would)
         if g_a is None and g_at is None:
             need[5] = need[8] = need[9] = False                             # the map l, gamma, beta
@@ -940,12 +979,12 @@ class _PainnUpdate(torch.autograd.Function):
         g_a, g_v = zeros(g_a, x_a), zeros(g_v, x_v)
         if x_vt is not None:
             g_at, g_vt = zeros(g_at, x_a), zeros(g_vt, x_v)
-        g_x, d_params = ops.painn_update_train_bwd(g_a, g_at, g_v, g_vt, params[5::2], upd.gn.groups, params[3], rows)
+        g_x, d_params = ops.painn_update_train_bwd(g_a, g_at, g_v, g_vt, params[5::2], upd.gn.groups, params[3], rows, residual)
         grads = list(g_x) + list(d_params)
-        return (None,) + tuple(g if nd else None for g, nd in zip(grads, need[1:]))
+        return (None, None) + tuple(g if nd else None for g, nd in zip(grads, need[1:]))
 
 
-def _update_pieces(upd, params, x_a, x_v, maps=None):
+def _update_pieces(upd, params, x_a, x_v, maps=None, residual=False):
     """painn.Update out of differentiable pieces; params: gamma, beta and the MLP's behind the three maps' weights, which
     `maps` (callables) stand in for."""
     n = upd.n
@@ -956,23 +995,24 @@ def _update_pieces(upd, params, x_a, x_v, maps=None):
     y = _mlp_rows(params[-6:], torch.cat([x_a, torch.linalg.vector_norm(v_r, dim=-1)], dim=-1))
     v = lin_v(x_v) * y[..., :n, None]
     a = scal_group_norm(upd.gn, ip * y[..., n:2 * n], params[-8], params[-7]) + y[..., 2 * n:]
-    return a, v / torch.sqrt(add((v ** 2).sum(-1, keepdim=True), 1.))
+    v = v / torch.sqrt(add((v ** 2).sum(-1, keepdim=True), 1.))
+    return (add(x_a, a), add(x_v, v)) if residual else (a, v)
 
 
-def painn_update(upd, x_a, x_v):
-    """archs/meanflow_painn8.py:63-75"""
+def painn_update(upd, x_a, x_v, residual=False):
+    """archs/meanflow_painn8.py:63-75; (x_a + da, x_v + dv) with residual, as painn_message."""
     maps = (upd.lin_l, upd.lin_r, upd.lin_v)
     params = [upd.gn.gamma, upd.gn.beta, *_mlp_parameters(upd.mlp)]
     if not all(plain_call(lin, TensLinear) for lin in maps):
-        return _update_pieces(upd, params, x_a, x_v, maps)
+        return _update_pieces(upd, params, x_a, x_v, maps, residual)
     params = [lin.W for lin in maps] + params
     pairs = [tuple(_dense(t) for t in _unpack(x)) for x in (x_a, x_v)]
     (a, a_t), (v, v_t) = pairs
     if a_t is not None and v_t is None:
         v_t = torch.zeros_like(v)
     if not (x_a.dim() == 3 and upd.n <= 256 and _fused(params, a, a_t, v, v_t)):
-        return _update_pieces(upd, params, x_a, x_v)
-    outs = _PainnUpdate.apply(upd, a, a_t, v, v_t, *params)
+        return _update_pieces(upd, params, x_a, x_v, residual=residual)
+    outs = _PainnUpdate.apply(upd, residual, a, a_t, v, v_t, *params)
     return outs if v_t is None else tuple(fwAD.make_dual(p, t) for p, t in zip(outs[:2], outs[2:]))
 
 

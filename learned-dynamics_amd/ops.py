@@ -1240,24 +1240,29 @@ mlp_silu_bwd = _ext.mlp_silu_bwd
 mlp_leaky_takes, mlp_leaky_fwd, mlp_leaky_bwd = _ext.mlp_leaky_takes, _ext.mlp_leaky_fwd, _ext.mlp_leaky_bwd
 painn_edge_encode_fwd = _ext.edge_encode_fwd
 painn_edge_encode_bwd = _ext.edge_encode_bwd
-painn_combine_dual_bwd = _ext.combine_dual_bwd
 
 
 def painn_grid_message_bwd(table, actv, actv_sliced, v, r_ij, g_v, g_a, src, dst, row_ptr, order, node_order, period, epsilon,
-                           want_table, want_actv, want_v, src_row_ptr=None):
+                           want_table, want_actv, want_v, src_row_ptr=None, residual=False):
     """(d_table, d_actv, d_v) of the message interpolated from its grid.  src_row_ptr: rows of the edges by source; with node_order
-    the grid's gradient then takes the edges in that order of their sources."""
+    the grid's gradient then takes the edges in that order of their sources.  residual: v was added to out_v, and d_v is the sum
+    of both gradients."""
     return _ext.painn_grid_message_bwd(table, actv, actv_sliced, v, r_ij, g_v, g_a, src, dst, row_ptr, order, node_order, period,
-                                       epsilon, bool(want_table), bool(want_actv), bool(want_v), src_row_ptr)
+                                       epsilon, bool(want_table), bool(want_actv), bool(want_v), src_row_ptr, bool(residual))
 
 
 painn_update_train_fwd = _ext.painn_update_train_fwd
 painn_update_train_bwd = _ext.painn_update_train_bwd
 
 
-def painn_combine_dual_fwd(args, node, row_ptr, n_out):
-    """(dist, dist_t, actv, actv_t, v, v_t, direction, direction_t), tangents or None -> (out_v, out_a, out_v_t, out_a_t)."""
-    return tuple(_ext.combine_dual_fwd(args, node, row_ptr, n_out))
+def painn_combine_dual_bwd(args, row_ptr, order, grads, grad_row, n_grad_rows, want, residual=False):
+    return _ext.combine_dual_bwd(args, row_ptr, order, grads, grad_row, n_grad_rows, want, residual)
+
+
+def painn_combine_dual_fwd(args, node, row_ptr, n_out, residual=()):
+    """(dist, dist_t, actv, actv_t, v, v_t, direction, direction_t), tangents or None -> (out_v, out_a, out_v_t, out_a_t).
+    residual: (a, a_t, v, v_t), any None, added to the results."""
+    return tuple(_ext.combine_dual_fwd(args, node, row_ptr, n_out, list(residual)))
 
 
 # ------------------------------------------------- bf16-storage configuration

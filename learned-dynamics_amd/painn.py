@@ -162,8 +162,7 @@ class Update(nn.Module):
     def forward(self, x_a, x_v, residual=False):
         """Returns (dx_a, dx_v), or (x_a + dx_a, x_v + dx_v) with residual=True."""
         if diff.wants_grad(self, x_a, x_v):
-            da, dv = diff.painn_update(self, x_a, x_v)
-            return (diff.add(x_a, da), diff.add(x_v, dv)) if residual else (da, dv)
+            return diff.painn_update(self, x_a, x_v, residual)
         params = (self.lin_l.W, self.lin_r.W, self.lin_v.W)
         cache = self.__dict__.setdefault("_lrv_cache", {})
         stamp = ops.stamp(params)
@@ -387,8 +386,7 @@ class Message(nn.Module):
         (filter_table of the rows that _grid_rows names), filters: the filter of every edge where no grid is read, if the
         caller has it already."""
         if diff.wants_grad(self, x_a, x_v, r_ij):
-            da, dv = diff.painn_message(self, graph, x_a, x_v, r_ij)
-            return (diff.add(x_a, da), diff.add(x_v, dv)) if residual else (da, dv)
+            return diff.painn_message(self, graph, x_a, x_v, r_ij, residual)
         B, N, n = x_a.shape
         x_a, x_v, r_ij = x_a.contiguous(), x_v.contiguous(), r_ij.contiguous()
         E = r_ij.shape[0]

@@ -1460,10 +1460,12 @@ def test_tensor_norm_and_its_adjoint_as_kernels(pkg, inds, chan, groups, batch, 
     assert torch.equal(torch.autograd.grad(norm(strided), strided, dy)[0], got[0])
 
 
+@pytest.mark.parametrize("residual", [False, True])
 @pytest.mark.parametrize("E,n,missing", [(1, 4, ()), (700, 128, ()), (701, 64, ("dist", "dir")), (90, 256, ("actv", "v"))])
-def test_messages_with_tangents_two_or_four_channels_a_lane(pkg, E, n, missing):
+def test_messages_with_tangents_two_or_four_channels_a_lane(pkg, E, n, missing, residual):
     """Message sums and their tangents and the gradients of both against the formula in float64: a handful of float32 roundings a term,
-    in sums over the edges of a row.  Rows of no edge, of one, of many; tangents that are left out."""
+    in sums over the edges of a row.  Rows of no edge, of one, of many; tangents that are left out; the node's own row added to the
+    sums, whose gradient the adjoint adds."""
     diff = importlib.import_module("learned-dynamics_amd.differentiable")
     gl = importlib.import_module("learned-dynamics_amd.graph_layers")
     g = torch.Generator().manual_seed(E + n)
@@ -1473,20 +1475,23 @@ def test_messages_with_tangents_two_or_four_channels_a_lane(pkg, E, n, missing):
     graph = gl.Graph(src.cuda(), dst.cuda(), None, 1, N)
     shapes = dict(dist=(E, 4 * n), actv=(N, 4 * n), v=(N, n, 3), dir=(E, 3))
     pairs = {k: [torch.randn(s, generator=g, dtype=F64).float(), torch.randn(s, generator=g, dtype=F64).float()] for k, s in shapes.items()}
+    if residual:
+        pairs["x"] = [torch.randn(N, n, generator=g, dtype=F64).float(), torch.randn(N, n, generator=g, dtype=F64).float()]
     for k in missing:
         pairs[k][1] = None
     flat = [t for p in pairs.values() for t in p]
     cpu = [None if t is None else t.double().requires_grad_() for t in flat]
     gpu = [None if t is None else t.cuda().requires_grad_() for t in flat]
 
-    def sums(dist, actv, v, direction):
+    def sums(dist, actv, v, direction, x=None):
         m, a = diff._painn_combine_plain(dist, actv[dst], v[dst], direction)
-        return torch.zeros(N, n, 3, dtype=F64).index_add(0, src, m), torch.zeros(N, n, dtype=F64).index_add(0, src, a)
+        first = (v, x) if residual else (torch.zeros(N, n, 3, dtype=F64), torch.zeros(N, n, dtype=F64))
+        return first[0].index_add(0, src, m), first[1].index_add(0, src, a)
 
     values, tangents = tuple(cpu[0::2]), tuple(torch.zeros_like(c) if t is None else t for c, t in zip(cpu[0::2], cpu[1::2]))
     ref, ref_t = torch.autograd.functional.jvp(sums, values, tangents, create_graph=True)
     want = (*ref, *ref_t)
-    got = diff._PainnCombineDual.apply(graph.by_dst, graph.by_src, *gpu)
+    got = diff._PainnCombineDual.apply(graph.by_dst, graph.by_src, *(gpu[8:] or (None, None)), *gpu[:8])
     weights = [torch.randn(w.shape, generator=g, dtype=F64).float() for w in want]
     live = [i for i, t in enumerate(gpu) if t is not None]
     g_want = torch.autograd.grad(sum((w * k.double()).sum() for w, k in zip(want, weights)), [cpu[i] for i in live])
@@ -1516,3 +1521,44 @@ def test_row_pointers_of_long_runs_of_empty_rows(ops, dtype):
         index = torch.tensor(rows, dtype=dtype)
         want = torch.searchsorted(index, torch.arange(n + 1, dtype=dtype))
         assert torch.equal(ops.segment_row_ptr(index.cuda(), n).cpu().long(), want), (rows[:4], n)
+
+
+@pytest.mark.parametrize("E,n", [(30000, 64), (600, 64), (600, 24)])
+def test_layers_that_add_their_input(pkg, E, n):
+    """Message and Update of training with residual=True against the same layers with the input added outside: filters from their
+    grid, from the MLP on every edge, and in pieces (n no power of two); values, values with tangents, gradients, recorded gradients.
+    The additions are the same ones: results to a rounding, gradients to the order in which two of their terms are added."""
+    painn = importlib.import_module("learned-dynamics_amd.painn")
+    gl = importlib.import_module("learned-dynamics_amd.graph_layers")
+    diff = importlib.import_module("learned-dynamics_amd.differentiable")
+    g = torch.Generator().manual_seed(E + n)
+    torch.manual_seed(n)
+    N = 300
+    src = torch.sort(torch.randint(0, N, (E,), generator=g)).values
+    dst = torch.randint(0, N, (E,), generator=g)
+    graph = gl.Graph(src.cuda(), dst.cuda(), None, 1, N)
+    message, update = painn.Message(5.0, n).cuda(), painn.Update(n).cuda()
+    r = torch.randn(E, 3, generator=g).cuda()
+    x_a, x_v, t_a, t_v = (torch.randn(*s, generator=g).cuda() for s in [(1, N, n), (1, N, n, 3)] * 2)
+    x_a, x_v = x_a.requires_grad_(), x_v.requires_grad_()
+    w = [torch.randn(1, N, n, generator=g).cuda(), torch.randn(1, N, n, 3, generator=g).cuda()]
+
+    def outside(f):
+        return lambda a, v: tuple(diff.add(x, d) for x, d in zip((a, v), f(a, v, False)))
+
+    for layer in (lambda a, v, res: message(graph, a, v, r, residual=res), lambda a, v, res: update(a, v, residual=res)):
+        inside = lambda a, v: layer(a, v, True)
+        ways = []
+        for f in (outside(layer), inside):
+            out = f(x_a, x_v)
+            first = torch.autograd.grad(out, (x_a, x_v), w, retain_graph=True)
+            recorded = torch.autograd.grad(out, (x_a, x_v), w, create_graph=True)
+            value, tangent = diff.jvp(f, (x_a, x_v), (t_a, t_v))
+            both = torch.autograd.grad((*value, *tangent), (x_a, x_v), w + w)
+            only_a = torch.autograd.grad(f(x_a, x_v)[0].sum(), (x_a, x_v), allow_unused=True)
+            ways.append([*out, *first, *recorded, *value, *tangent, *both, *only_a])
+        for k, (a, b) in enumerate(zip(*ways)):
+            assert (a is None) == (b is None), k
+            if a is not None:
+                err, size = float((a.detach() - b.detach()).norm()), float(a.detach().norm())
+                assert err <= 2e-6 * size, (k, err, size)
