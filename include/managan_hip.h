@@ -481,6 +481,21 @@ int mg_tensor_linear_wgrad_f16x2_rows(const float* dy, const float* x, const flo
 int mg_tensor_linear_wgrad_f16x2_groups(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,
                                         const float* x_rowmax, int groups, long rows, int dim_in, int dim_out, void* workspace,
                                         float* dW, mg_stream_t stream);
+/* Several of them over the same rows, as few launches as their sizes allow (the weight gradients of an MLP's layers).  db NULL: not
+ * wanted; a bound NULL: taken from the data.  workspace: mg_tensor_linear_wgrad_f16x2_many_workspace_bytes of the same jobs. */
+#define MG_WGRAD_F16X2_JOBS 4      /* products of one launch at most */
+typedef struct mg_wgrad_f16x2 {
+    const float *dy, *x, *dy_bound;
+    long n_dy_bound;
+    const float* x_bound;
+    long n_x_bound, bias_rows;
+    int dim_in, dim_out;
+    float *dW, *db;
+} mg_wgrad_f16x2;
+int mg_tensor_linear_wgrad_f16x2_many_workspace_bytes(const mg_wgrad_f16x2* jobs /* host */, int count, long rows,
+                                                      size_t* bytes /* host */);
+int mg_tensor_linear_wgrad_f16x2_many(const mg_wgrad_f16x2* jobs /* host */, int count, long rows, void* workspace,
+                                      mg_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Ant16 (managan/codegen_tensor_products.py:19-34; ant16_o0_cuda / ant16_o1_cuda / ant16_o2_cuda /

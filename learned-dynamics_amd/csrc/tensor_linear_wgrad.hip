@@ -305,20 +305,26 @@ __global__ void __launch_bounds__(256) absmax_parts_kernel(const float* __restri
     __syncthreads();
     if (threadIdx.x == 0) parts[blockIdx.x] = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
 }
-// the same for one or two arrays of any length and alignment (bounds handed in by the caller) in one launch: the first
-// blocks_a workgroups take the first array
+// the same for several arrays of any length and alignment (bounds handed in by the caller) in one launch: array k from workgroup
+// first_block on
 struct BoundArray {
     const float* data;
     long n;
     float* parts;
-    int blocks;
+    int blocks, first_block;
 };
-__global__ void __launch_bounds__(256) absmax_parts_scalar_kernel(const BoundArray a, const BoundArray b) {
-    const bool first = (int)blockIdx.x < a.blocks;
-    const float* __restrict__ x = first ? a.data : b.data;
-    const long n = first ? a.n : b.n, stride = 256L * (first ? a.blocks : b.blocks);
-    const int block = first ? blockIdx.x : blockIdx.x - a.blocks;
-    float* __restrict__ parts = first ? a.parts : b.parts;
+struct BoundArrays {
+    BoundArray array[2 * MG_WGRAD_F16X2_JOBS];
+    int count;
+};
+__global__ void __launch_bounds__(256) absmax_parts_scalar_kernel(const BoundArrays arrays) {
+    int which = 0;
+    while (which + 1 < arrays.count && (int)blockIdx.x >= arrays.array[which + 1].first_block) which++;     // (uniform)
+    const BoundArray& a = arrays.array[which];
+    const float* __restrict__ x = a.data;
+    const long n = a.n, stride = 256L * a.blocks;
+    const int block = blockIdx.x - a.first_block;
+    float* __restrict__ parts = a.parts;
     float m = 0.f;
     for (long k = (long)block * 256 + threadIdx.x; k < n; k += stride) m = fmaxf(m, fabsf(x[k]));
     for (int d = 1; d < 64; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
@@ -338,25 +344,42 @@ __global__ void __launch_bounds__(256) absmax_columns_kernel(const float* __rest
     if (threadIdx.x == 0) parts[blockIdx.y * gridDim.x + blockIdx.x] = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
 }
 
-// group_cols: columns of x that share a scale (I: all of them)
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) wgrad_f16x2_kernel(const float* __restrict__ dy, const float* __restrict__ x,
-                                                          const float* __restrict__ dy_parts, int n_dy_parts,
-                                                          const float* __restrict__ x_parts, int n_x_parts, int group_cols,
-                                                          long R, int I, int O, long rows_per_block,
-                                                          float* __restrict__ part, float* __restrict__ colsum_part,
-                                                          long bias_rows) {
+// One product dW = dy^T x of several over the same R rows.  group_cols: columns of x that share a scale (I: all of them); part: where
+// its partial sums lie in the plane of a slice; colsum: the same of the column sums of dy, or negative.
+struct WgradJob {
+    const float *dy, *x, *dy_parts, *x_parts;
+    int n_dy_parts, n_x_parts, group_cols, I, O, first_tile;
+    long part, colsum, bias_rows;
+};
+struct WgradJobs {
+    WgradJob job[MG_WGRAD_F16X2_JOBS];
+    int count, tiles;
+    long R, rows_per_block, plane;                         // plane: floats of a slice
+    float* parts;
+};
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) wgrad_f16x2_kernel(const WgradJobs jobs) {
     // [stage buffer][operand: dy, x][piece: hi, lo][LDS row][64 bytes]
     __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kFBuf];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m = lane & 31, g = lane >> 5;
     // Workgroup ids go round-robin over the 8 XCDs: XCD x takes the x-th eighth of the (slice, tile) pairs, slice by slice, so that the
     // tiles of a slice, which read the same rows four times over, find them in one L2
-    const int tiles_o = (int)ceil_div(O, kFTile), tiles = tiles_o * (int)ceil_div(I, kFTile);
+    // (the tiles of all products that a launch takes)
+    const long R = jobs.R, rows_per_block = jobs.rows_per_block;
+    const int tiles = jobs.tiles;
     const long slices = ceil_div(R, rows_per_block), per_xcd = ceil_div(slices * tiles, 8);
     const long item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if ((blockIdx.x >> 3) >= per_xcd || item >= slices * tiles) return;
     const long slice = item / tiles;
-    const int tile = (int)(item - slice * tiles), o_tile = tile % tiles_o * kFTile, i_tile = tile / tiles_o * kFTile;
+    const int all_tile = (int)(item - slice * tiles);
+    int which = 0;
+    while (which + 1 < jobs.count && all_tile >= jobs.job[which + 1].first_tile) which++;     // (uniform)
+    const WgradJob& job = jobs.job[which];
+    const float *__restrict__ dy = job.dy, *__restrict__ x = job.x, *__restrict__ dy_parts = job.dy_parts, *__restrict__ x_parts = job.x_parts;
+    const int n_dy_parts = job.n_dy_parts, n_x_parts = job.n_x_parts, group_cols = job.group_cols, I = job.I, O = job.O;
+    const long bias_rows = job.bias_rows;
+    const int tile = all_tile - job.first_tile, tiles_o = (int)ceil_div(O, kFTile);
+    const int o_tile = tile % tiles_o * kFTile, i_tile = tile / tiles_o * kFTile;
     const long r_lo = slice * rows_per_block;
     const long r_hi = r_lo + rows_per_block < R ? r_lo + rows_per_block : R;
 
@@ -382,7 +405,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int u = 0; u < 8; u++) v[u] = *reinterpret_cast<const float4*>(rows + u * dim + lane_off);
     };
     // column sums of dy over the slice (the bias gradient), by the workgroups of the first column of tiles
-    const bool sum_cols = colsum_part != nullptr && i_tile == 0;                   // (uniform)
+    const bool sum_cols = job.colsum >= 0 && i_tile == 0;                          // (uniform)
     float4 colsum = make_float4(0.f, 0.f, 0.f, 0.f);
     // One stage in eight parts: part g splits columns 2 (g % 2) and one more of rows 2 (g / 2) and one more of the stage at r, which
     // are in v or on their way there; every second part requests the same two rows of the stage at r_next.  finish writes the pieces.
@@ -556,7 +579,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     set_scales();                                          // (the first stage is on its way meanwhile)
     if (sum_cols) walk(std::true_type{});
     else walk(std::false_type{});
-    if (colsum_part != nullptr && i_tile == 0) {                              // (uniform)
+    float* plane = jobs.parts + slice * jobs.plane;
+    if (sum_cols) {
         // the four row groups of a column quad, added in a fixed order
         float4* sums = reinterpret_cast<float4*>(lds);                             // [octet][cq]; the stage buffers are done with
         if (!stage_x) sums[octet * 32 + cq] = colsum;
@@ -565,24 +589,22 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
             const float4 s0 = sums[cq], s1 = sums[32 + cq], s2 = sums[64 + cq], s3 = sums[96 + cq];
             const int o = o_tile + 4 * cq;
             if (o < O)
-                *reinterpret_cast<float4*>(colsum_part + slice * O + o) =
+                *reinterpret_cast<float4*>(plane + job.colsum + o) =
                     make_float4((s0.x + s1.x) + (s2.x + s3.x), (s0.y + s1.y) + (s2.y + s3.y),
                                 (s0.z + s1.z) + (s2.z + s3.z), (s0.w + s1.w) + (s2.w + s3.w));
         }
     }
     // D[row][col]: col = lane % 32, row = 8 (k / 4) + 4 (lane / 32) + k % 4 for register k; LDS row 32 j + c / 4 of
     // an operand is column 4 (c / 4) + j of the tile
-    float* plane = part + slice * O * I;
+    float* out = plane + job.part;
+    const int i = i_tile + 4 * m + 2 * (wave & 1);         // (and i + 1: I is a multiple of four)
 #pragma unroll
     for (int p = 0; p < 2; p++)
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const int i = i_tile + 4 * m + 2 * (wave & 1) + q;
-#pragma unroll
-            for (int k = 0; k < 16; k++) {
-                const int o = o_tile + 4 * (8 * (k / 4) + 4 * g + (k % 4)) + 2 * (wave >> 1) + p;
-                if (o < O && i < I) plane[(long)o * I + i] = total[p][q][k] * unscale[q];
-            }
+        for (int k = 0; k < 16; k++) {
+            const int o = o_tile + 4 * (8 * (k / 4) + 4 * g + (k % 4)) + 2 * (wave >> 1) + p;
+            if (o < O && i < I)
+                *reinterpret_cast<float2*>(out + (long)o * I + i) = make_float2(total[p][0][k] * unscale[0], total[p][1][k] * unscale[1]);
         }
 }
 
@@ -604,36 +626,43 @@ __global__ void __launch_bounds__(256) wgrad_reduce_kernel(const float* __restri
     }
 }
 
-// the same for two sets of planes in one launch (the weight gradient and the column sums)
-__global__ void __launch_bounds__(256) wgrad_reduce2_kernel(const float* __restrict__ part_a, long n_a,
-                                                            float* __restrict__ out_a,
-                                                            const float* __restrict__ part_b, long n_b,
-                                                            float* __restrict__ out_b, int splits) {
-    for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < n_a + n_b; k += (long)gridDim.x * blockDim.x) {
-        const bool first = k < n_a;
-        const float* src = first ? part_a + k : part_b + (k - n_a);
-        const long stride = first ? n_a : n_b;
-        float s = 0.f;
-        int z = 0;
-        for (; z + 8 <= splits; z += 8) {                  // eight loads in flight, added in slice order
-            float v[8];
+// the same for the planes of several products: quad k of a plane goes to the segment that holds it
+struct WgradSegments {
+    float* out[2 * MG_WGRAD_F16X2_JOBS];
+    int first_quad[2 * MG_WGRAD_F16X2_JOBS];
+    int count;
+    bool aligned;                                          // every out is 16-byte aligned
+};
+__global__ void __launch_bounds__(256) wgrad_reduce_f16x2_kernel(const float4* __restrict__ part, int quads, int splits,
+                                                                 const WgradSegments seg) {
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    if (k >= quads) return;
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto add = [&](const float4& v) { s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w; };
+    int z = 0;
+    for (; z + 8 <= splits; z += 8) {                      // eight loads in flight, added in slice order
+        float4 v[8];
 #pragma unroll
-            for (int u = 0; u < 8; u++) v[u] = src[(long)(z + u) * stride];
+        for (int u = 0; u < 8; u++) v[u] = part[(long)(z + u) * quads + k];
 #pragma unroll
-            for (int u = 0; u < 8; u++) s += v[u];
-        }
-        for (; z < splits; z++) s += src[(long)z * stride];
-        if (first) out_a[k] = s; else out_b[k - n_a] = s;
+        for (int u = 0; u < 8; u++) add(v[u]);
     }
+    for (; z < splits; z++) add(part[(long)z * quads + k]);
+    float* out = seg.out[0];
+    int first = 0;
+#pragma unroll
+    for (int j = 1; j < 2 * MG_WGRAD_F16X2_JOBS; j++)
+        if (j < seg.count && k >= seg.first_quad[j]) { out = seg.out[j]; first = seg.first_quad[j]; }
+    out += 4L * (k - first);
+    if (seg.aligned) *reinterpret_cast<float4*>(out) = s;
+    else { out[0] = s.x; out[1] = s.y; out[2] = s.z; out[3] = s.w; }
 }
 
 // rows per slice and number of slices for a problem (the same on the sizing and the launching side)
 // resident_groups = 0: aim at ~4 workgroups per CU; otherwise the number of workgroups the chip holds at once, which
 // the grid then does not exceed (a second, partly filled round would cost a whole slice's time)
-void wgrad_split(long rows, int dim_in, int dim_out, int tile, long* rows_per_block, long* splits,
-                 long resident_groups = 0) {
-    const int gx = (int)ceil_div(dim_out, tile), gy = (int)ceil_div(dim_in, tile);
-    long s = resident_groups > 0 ? resident_groups / ((long)gx * gy) : ceil_div(1024, (long)gx * gy);
+void wgrad_split_tiles(long rows, long tiles, long* rows_per_block, long* splits, long resident_groups = 0) {
+    long s = resident_groups > 0 ? resident_groups / tiles : ceil_div(1024, tiles);
     const long max_splits = ceil_div(rows, 64);
     if (s > max_splits) s = max_splits;
     if (s < 1) s = 1;
@@ -642,6 +671,9 @@ void wgrad_split(long rows, int dim_in, int dim_out, int tile, long* rows_per_bl
     rpb = ceil_div(rpb, 32) * 32;                      // (a multiple of every kernel's rows per trip)
     *rows_per_block = rpb;
     *splits = rows > 0 ? ceil_div(rows, rpb) : 0;
+}
+void wgrad_split(long rows, int dim_in, int dim_out, int tile, long* rows_per_block, long* splits) {
+    wgrad_split_tiles(rows, ceil_div(dim_out, tile) * ceil_div(dim_in, tile), rows_per_block, splits);
 }
 // plain rows take the matrix-core kernel and its 128 x 128 tiles
 inline int wgrad_tile(int inds) { return inds == 0 ? kMTile : kTile; }
@@ -669,67 +701,163 @@ int mg_tensor_linear_wgrad_f16x2_supported(long rows, int dim_in, int dim_out) {
     return rows >= 4096 && dim_in >= 4 && dim_out >= 4 && dim_in % 4 == 0 && dim_out % 4 == 0;
 }
 
-// groups > 1: x_bound holds (rows, groups) maxima, one of each dim_in / groups columns
-static int wgrad_f16x2(const float* dy, const float* x, const float* dy_bound, long n_dy_bound, const float* x_bound, long n_x_bound,
-                       int groups, long rows, long bias_rows, int dim_in, int dim_out, void* workspace, float* dW, float* db,
-                       mg_stream_t stream) {
-    MG_REQUIRE(mg_tensor_linear_wgrad_f16x2_supported(rows, dim_in, dim_out),
-               "mg_tensor_linear_wgrad_f16x2: needs rows >= 4096 and dims that are multiples of 4");
-    MG_REQUIRE(dy && x && workspace && dW, "mg_tensor_linear_wgrad_f16x2: null pointer");
-    MG_REQUIRE(aligned16(dy) && aligned16(x), "mg_tensor_linear_wgrad_f16x2: dy and x must be 16-byte aligned");
-    MG_REQUIRE((dy_bound == nullptr || n_dy_bound > 0) && (x_bound == nullptr || n_x_bound > 0),
-               "mg_tensor_linear_wgrad_f16x2: empty bound array");
+// How many of the first of `count` products over the same rows go together: while their tiles leave the chip's 256 compute units two
+// slices.  What a launch costs beside its products, the bounds that every workgroup reads, the first loads, the partial results of
+// as many workgroups as the chip holds and their sum, is then paid once, and the slices are longer: the three products of
+// an MLP 128 -> 512 -> 512 -> 512 at 4096 rows 77 -> 39 us, at 8192 92 -> 56, at 32 768 242 -> 183, at 155 744 806 -> 758; four of
+// 256 x 256 at 24 576 141 -> 76; 512 x 1024 and two of 1024 x 1024 at 8192 (two launches) 204 -> 194.  Errors against float64 are those of
+// single products or less.
+constexpr long kMergedTiles = 128;
+static long job_tiles(const mg_wgrad_f16x2& j) { return ceil_div(j.dim_out, kFTile) * ceil_div(j.dim_in, kFTile); }
+static int together(const mg_wgrad_f16x2* jobs, int count) {
+    long tiles = 0;
+    for (int k = 0; k < count && k < MG_WGRAD_F16X2_JOBS; k++) {
+        tiles += job_tiles(jobs[k]);
+        if (k > 0 && tiles > kMergedTiles) return k;
+    }
+    return count < MG_WGRAD_F16X2_JOBS ? count : MG_WGRAD_F16X2_JOBS;
+}
+static void slices_of(const mg_wgrad_f16x2* jobs, int count, long rows, long* rpb, long* splits, long* plane) {
+    long tiles = 0;
+    *plane = 0;
+    for (int k = 0; k < count; k++) {
+        tiles += job_tiles(jobs[k]);
+        *plane += (long)jobs[k].dim_in * jobs[k].dim_out + (jobs[k].db ? jobs[k].dim_out : 0);
+    }
+    // Two workgroups per CU fit; where that leaves slices of fewer than some 320 rows, one per CU is faster (half the partial results to
+    // write and add up; one against two: 4096 x 512 x 512 29, 35 us, four of 64 x 64 at 8192 19, 24, 64 x 256 and two of 256 x 256 at
+    // 8192 28, 30; but 256 x 384 and two of 384 x 384 at 8192 47, 43, at 16 384 78, 70, 101 000 x 512 x 512 281, 238)
+    constexpr long kShortSlices = 163840;
+    wgrad_split_tiles(rows, tiles, rpb, splits, rows < 65536 && rows * tiles < kShortSlices ? 256 : 512);
+}
+
+// x_groups > 1: x_bound holds (rows, x_groups) maxima, one of each dim_in / x_groups columns
+static int wgrad_f16x2(const mg_wgrad_f16x2* jobs, int count, int x_groups, long rows, void* workspace, mg_stream_t stream) {
     hipStream_t st = (hipStream_t)stream;
-    const long n = (long)dim_in * dim_out;
-    long rpb, splits;
-    // two workgroups per CU fit; with node-sized operands one per CU is faster (longer slices, half the partial
-    // results to write and add up: 4096 x 512 x 512 29 against 35 us, 12288 x 128 x 384 26 against 30 us;
-    // 101000 x 512 x 512 281 against 238 us)
-    wgrad_split(rows, dim_in, dim_out, kFTile, &rpb, &splits, rows < 65536 ? 256 : 512);
-    float* part = reinterpret_cast<float*>((reinterpret_cast<uintptr_t>(workspace) + 15) & ~uintptr_t(15));
-    float* maxima = part + splits * n;                       // [dy: kFParts][x: kFParts]
-    float* colsum_part = db ? maxima + 2 * kFParts : nullptr; // [slice][dim_out]
+    WgradJobs all{};
+    long rpb, splits, plane;
+    slices_of(jobs, count, rows, &rpb, &splits, &plane);
+    all.count = count;
+    all.R = rows;
+    all.rows_per_block = rpb;
+    all.plane = plane;
+    all.parts = reinterpret_cast<float*>((reinterpret_cast<uintptr_t>(workspace) + 15) & ~uintptr_t(15));
+    float* maxima = all.parts + splits * plane;              // per job [dy: kFParts][x: kFParts]
     constexpr long kDirectBounds = 16384;                    // a bound array this short is read by every workgroup itself
     auto blocks_for = [](long len) { return (int)(ceil_div(len, 4096) < kFParts ? ceil_div(len, 4096) : kFParts); };
-    BoundArray scan[2] = {};
-    // partial maxima of the caller's bounds, or of the data itself
-    auto bound_parts = [&](BoundArray& a, const float* data, long count, const float* bound, long n_bound, float* parts) -> int {
+    BoundArrays scan{};
+    int scan_blocks = 0;
+    // partial maxima of the caller's bounds, or of the data itself; an array that two products share is scanned once
+    auto bound_parts = [&](const float* data, long n_data, const float* bound, long n_bound, float* parts, const float** from) -> int {
+        *from = bound;
         if (bound && n_bound <= kDirectBounds) return (int)n_bound;
-        const int blocks = blocks_for(bound ? n_bound : count);
-        if (bound) a = BoundArray{bound, n_bound, parts, blocks};
-        else hipLaunchKernelGGL(absmax_parts_kernel, dim3(blocks), dim3(256), 0, st, data, count, parts);
+        *from = parts;
+        const int blocks = blocks_for(bound ? n_bound : n_data);
+        if (!bound) {
+            hipLaunchKernelGGL(absmax_parts_kernel, dim3(blocks), dim3(256), 0, st, data, n_data, parts);
+            return blocks;
+        }
+        for (int k = 0; k < scan.count; k++)
+            if (scan.array[k].data == bound && scan.array[k].n == n_bound) {
+                *from = scan.array[k].parts;
+                return blocks;
+            }
+        scan.array[scan.count++] = BoundArray{bound, n_bound, parts, blocks, scan_blocks};
+        scan_blocks += blocks;
         return blocks;
     };
-    const int na = bound_parts(scan[0], dy, rows * dim_out, dy_bound, n_dy_bound, maxima);
-    int nb;
-    if (groups > 1) {
-        const long per = kFParts / groups;
-        nb = (int)(ceil_div(rows, 1024) < per ? ceil_div(rows, 1024) : per);
-        hipLaunchKernelGGL(absmax_columns_kernel, dim3((unsigned)nb, (unsigned)groups), dim3(256), 0, st, x_bound, rows, groups, maxima + kFParts);
-    } else {
-        nb = bound_parts(scan[1], x, rows * dim_in, x_bound, n_x_bound, maxima + kFParts);
+    WgradSegments seg{};
+    seg.aligned = true;
+    long at = 0;
+    auto segment = [&](float* out, long n) {
+        seg.out[seg.count] = out;
+        seg.first_quad[seg.count++] = (int)(at / 4);
+        seg.aligned = seg.aligned && aligned16(out);
+        at += n;
+        return at - n;
+    };
+    for (int k = 0; k < count; k++) {
+        const mg_wgrad_f16x2& j = jobs[k];
+        WgradJob& to = all.job[k];
+        to = WgradJob{j.dy, j.x, nullptr, nullptr, 0, 0, j.dim_in / x_groups, j.dim_in, j.dim_out, all.tiles, 0, -1, j.bias_rows};
+        all.tiles += (int)job_tiles(j);
+        float *dy_maxima = maxima + 2L * k * kFParts, *x_maxima = dy_maxima + kFParts;
+        to.n_dy_parts = bound_parts(j.dy, rows * j.dim_out, j.dy_bound, j.n_dy_bound, dy_maxima, &to.dy_parts);
+        if (x_groups > 1) {
+            const long per = kFParts / x_groups;
+            to.n_x_parts = (int)(ceil_div(rows, 1024) < per ? ceil_div(rows, 1024) : per);
+            to.x_parts = x_maxima;
+            hipLaunchKernelGGL(absmax_columns_kernel, dim3((unsigned)to.n_x_parts, (unsigned)x_groups), dim3(256), 0, st, j.x_bound, rows,
+                               x_groups, x_maxima);
+        } else {
+            to.n_x_parts = bound_parts(j.x, rows * j.dim_in, j.x_bound, j.n_x_bound, x_maxima, &to.x_parts);
+        }
+        to.part = segment(j.dW, (long)j.dim_in * j.dim_out);
     }
-    if (scan[0].blocks + scan[1].blocks > 0)
-        hipLaunchKernelGGL(absmax_parts_scalar_kernel, dim3((unsigned)(scan[0].blocks + scan[1].blocks)), dim3(256), 0, st, scan[0],
-                           scan[1]);
-    const float* dy_parts = (dy_bound && n_dy_bound <= kDirectBounds) ? dy_bound : maxima;
-    const float* x_parts = (groups == 1 && x_bound && n_x_bound <= kDirectBounds) ? x_bound : maxima + kFParts;
-    const long items = ceil_div(dim_out, kFTile) * ceil_div(dim_in, kFTile) * splits;
-    MG_REQUIRE(items < (1L << 31) - 8, "mg_tensor_linear_wgrad_f16x2: grid too large");
-    dim3 grid((unsigned)(8 * ceil_div(items, 8))), block(256);
-    hipLaunchKernelGGL(wgrad_f16x2_kernel, grid, block, 0, st, dy, x, dy_parts, na, x_parts, nb, dim_in / groups, rows, dim_in,
-                       dim_out, rpb, part, colsum_part, bias_rows);
-    const long n_sum = n + (db ? dim_out : 0);
-    const unsigned nblocks = (unsigned)(ceil_div(n_sum, 256) < 1024 ? ceil_div(n_sum, 256) : 1024);
-    hipLaunchKernelGGL(wgrad_reduce2_kernel, dim3(nblocks), dim3(256), 0, st, (const float*)part, n, dW,
-                       (const float*)colsum_part, (long)(db ? dim_out : 0), db, (int)splits);
+    for (int k = 0; k < count; k++)
+        if (jobs[k].db) all.job[k].colsum = segment(jobs[k].db, jobs[k].dim_out);
+    if (scan.count > 0) hipLaunchKernelGGL(absmax_parts_scalar_kernel, dim3((unsigned)scan_blocks), dim3(256), 0, st, scan);
+    const long items = all.tiles * splits;
+    MG_REQUIRE(items < (1L << 31) - 8 && plane / 4 < (1L << 31), "mg_tensor_linear_wgrad_f16x2: grid too large");
+    hipLaunchKernelGGL(wgrad_f16x2_kernel, dim3((unsigned)(8 * ceil_div(items, 8))), dim3(256), 0, st, all);
+    const int quads = (int)(plane / 4);
+    hipLaunchKernelGGL(wgrad_reduce_f16x2_kernel, dim3((unsigned)ceil_div(quads, 256)), dim3(256), 0, st,
+                       reinterpret_cast<const float4*>(all.parts), quads, (int)splits, seg);
     return check_launch("mg_tensor_linear_wgrad_f16x2");
+}
+
+static int check_jobs(const mg_wgrad_f16x2* jobs, int count, long rows) {
+    for (int k = 0; k < count; k++) {
+        const mg_wgrad_f16x2& j = jobs[k];
+        MG_REQUIRE(mg_tensor_linear_wgrad_f16x2_supported(rows, j.dim_in, j.dim_out),
+                   "mg_tensor_linear_wgrad_f16x2: needs rows >= 4096 and dims that are multiples of 4");
+        MG_REQUIRE(j.dy && j.x && j.dW, "mg_tensor_linear_wgrad_f16x2: null pointer");
+        MG_REQUIRE(aligned16(j.dy) && aligned16(j.x), "mg_tensor_linear_wgrad_f16x2: dy and x must be 16-byte aligned");
+        MG_REQUIRE((j.dy_bound == nullptr || j.n_dy_bound > 0) && (j.x_bound == nullptr || j.n_x_bound > 0),
+                   "mg_tensor_linear_wgrad_f16x2: empty bound array");
+    }
+    return MG_OK;
+}
+
+int mg_tensor_linear_wgrad_f16x2_many_workspace_bytes(const mg_wgrad_f16x2* jobs, int count, long rows, size_t* bytes) {
+    MG_REQUIRE(bytes != nullptr && count >= 0 && (jobs || count == 0) && rows >= 0,
+               "mg_tensor_linear_wgrad_f16x2_many_workspace_bytes: bad argument");
+    size_t most = 0;
+    for (int k = 0; k < count;) {
+        const int n = together(jobs + k, count - k);
+        long rpb, splits, plane;
+        slices_of(jobs + k, n, rows, &rpb, &splits, &plane);
+        const size_t need = ((size_t)splits * (size_t)plane + 2 * (size_t)n * kFParts) * sizeof(float) + 16;
+        most = need > most ? need : most;
+        k += n;
+    }
+    *bytes = most;
+    return MG_OK;
+}
+
+int mg_tensor_linear_wgrad_f16x2_many(const mg_wgrad_f16x2* jobs, int count, long rows, void* workspace, mg_stream_t stream) {
+    MG_REQUIRE(count >= 0 && (jobs || count == 0), "mg_tensor_linear_wgrad_f16x2_many: bad argument");
+    if (int code = check_jobs(jobs, count, rows)) return code;
+    MG_REQUIRE(workspace || count == 0, "mg_tensor_linear_wgrad_f16x2: null pointer");
+    for (int k = 0; k < count;) {
+        const int n = together(jobs + k, count - k);
+        if (int code = wgrad_f16x2(jobs + k, n, 1, rows, workspace, stream)) return code;
+        k += n;
+    }
+    return MG_OK;
+}
+
+static int wgrad_f16x2_one(const mg_wgrad_f16x2& job, int x_groups, long rows, void* workspace, mg_stream_t stream) {
+    if (int code = check_jobs(&job, 1, rows)) return code;
+    MG_REQUIRE(workspace, "mg_tensor_linear_wgrad_f16x2: null pointer");
+    return wgrad_f16x2(&job, 1, x_groups, rows, workspace, stream);
 }
 
 int mg_tensor_linear_wgrad_f16x2_rows(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,
                                       const float* x_bound, long n_x_bound, long rows, long bias_rows, int dim_in, int dim_out,
                                       void* workspace, float* dW, float* db, mg_stream_t stream) {
-    return wgrad_f16x2(dy, x, dy_bound, n_dy_bound, x_bound, n_x_bound, 1, rows, bias_rows, dim_in, dim_out, workspace, dW, db, stream);
+    return wgrad_f16x2_one({dy, x, dy_bound, n_dy_bound, x_bound, n_x_bound, bias_rows, dim_in, dim_out, dW, db}, 1, rows, workspace,
+                           stream);
 }
 
 int mg_tensor_linear_wgrad_f16x2_groups(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,
@@ -737,8 +865,8 @@ int mg_tensor_linear_wgrad_f16x2_groups(const float* dy, const float* x, const f
                                         float* dW, mg_stream_t stream) {
     MG_REQUIRE(groups >= 1 && groups <= kFParts && dim_in % (4 * groups) == 0 && x_rowmax,
                "mg_tensor_linear_wgrad_f16x2_groups: groups of a multiple of four columns, and their row maxima");
-    return wgrad_f16x2(dy, x, dy_bound, n_dy_bound, x_rowmax, rows * groups, groups, rows, rows, dim_in, dim_out, workspace, dW, nullptr,
-                       stream);
+    return wgrad_f16x2_one({dy, x, dy_bound, n_dy_bound, x_rowmax, rows * groups, rows, dim_in, dim_out, dW, nullptr}, groups, rows,
+                           workspace, stream);
 }
 
 int mg_tensor_linear_wgrad_f16x2(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,

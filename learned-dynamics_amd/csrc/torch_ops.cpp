@@ -1007,6 +1007,40 @@ std::pair<at::Tensor, OptTensor> rows_wgrad(const at::Tensor& dy, const at::Tens
     return {dW, want_bias ? OptTensor(dy.narrow(0, 0, bias_rows).sum(0)) : OptTensor()};
 }
 
+// rows_wgrad of several layers over the same rows
+struct RowsGradient {
+    at::Tensor dy, x;
+    bool want_bias;
+    OptTensor dy_bound, x_bound;
+};
+std::vector<std::pair<at::Tensor, OptTensor>> rows_wgrads(const std::vector<RowsGradient>& of, int64_t bias_rows) {
+    std::vector<std::pair<at::Tensor, OptTensor>> out;
+    bool merged = mg_get_linear_mode() == kModeF16x2;
+    for (const RowsGradient& g : of)
+        merged = merged && aligned16(g.x) && aligned16(g.dy) && g.x.size(0) == of[0].x.size(0) &&
+                 mg_tensor_linear_wgrad_f16x2_supported(g.x.size(0), (int)g.x.size(1), (int)g.dy.size(1));
+    if (!merged) {
+        for (const RowsGradient& g : of) out.push_back(rows_wgrad(g.dy, g.x, bias_rows, g.want_bias, g.dy_bound, g.x_bound));
+        return out;
+    }
+    std::vector<mg_wgrad_f16x2> jobs;
+    for (const RowsGradient& g : of) {
+        at::Tensor dW = floats(g.x, {g.dy.size(1), g.x.size(1)});
+        OptTensor db;
+        if (g.want_bias) db = floats(g.x, {g.dy.size(1)});
+        jobs.push_back({fp(g.dy), fp(g.x), fp(g.dy_bound), g.dy_bound.has_value() ? g.dy_bound->numel() : 0, fp(g.x_bound),
+                        g.x_bound.has_value() ? g.x_bound->numel() : 0, bias_rows, (int)g.x.size(1), (int)g.dy.size(1), fp(dW),
+                        db.has_value() ? fp(*db) : nullptr});
+        out.emplace_back(dW, db);
+    }
+    const int64_t rows = of[0].x.size(0);
+    size_t n = 0;
+    check(mg_tensor_linear_wgrad_f16x2_many_workspace_bytes(jobs.data(), (int)jobs.size(), rows, &n));
+    at::Tensor ws = bytes_like(of[0].x, n);
+    check(mg_tensor_linear_wgrad_f16x2_many(jobs.data(), (int)jobs.size(), rows, ws.data_ptr(), stream_of(of[0].x)));
+    return out;
+}
+
 // Wide layers on values and tangents together: the one kernel has one accumulator for the large products there, 2.75e-7 from
 // float64 where the split reductions of few rows are at 2.5e-7: it takes over where those end (4.1e-7 beyond).
 bool mlp_dual_takes(int64_t rows, const Tensors& W, bool dual) {
@@ -1107,8 +1141,15 @@ std::tuple<OptTensor, Tensors> mlp_rows_bwd(at::Tensor g, OptTensor g_bound, con
         a.dim_in = (int)S.size(1);
         a.dim = (int)dim;
         check(mg_mlp_f16x2_adjoint(&a, stream_of(g)));
-        weight_grads(2, g, g_bound);
-        for (int l = 1; l >= 0; l--) weight_grads(l, dz[l], OptTensor(m[l]));
+        if (want_params) {
+            const auto of = rows_wgrads({{dz[0], S, true, OptTensor(m[0]), saved[0]},
+                                         {dz[1], *saved[3], true, OptTensor(m[1]), saved[2]},
+                                         {g, *saved[6], true, g_bound, saved[5]}}, R);
+            for (int l = 0; l < 3; l++) {
+                params[2 * l] = of[l].first;
+                params[2 * l + 1] = *of[l].second;
+            }
+        }
         return {g_x, params};
     }
     for (int l = 2; l >= 0; l--) {
@@ -1234,15 +1275,13 @@ std::tuple<OptTensor, Tensors> mlp_leaky_bwd(const at::Tensor& g, const at::Tens
     if (want_x) run_f16x2(W[3].t(), W[3].size(0), fp(g), rows, Bound{OptTensor(g_max)}, OptTensor(), kActNone, true, 1, *g_x, nullptr, false);
     Tensors params;
     if (want_params) {
-        auto of = [&](const at::Tensor& dy, const at::Tensor& in, const at::Tensor& dy_bound, const at::Tensor& in_bound, bool bias) {
-            auto [dW, db] = rows_wgrad(dy, in, rows, bias, OptTensor(dy_bound), OptTensor(in_bound));
+        for (auto& [dW, db] : rows_wgrads({{dz[0], x, true, OptTensor(m[0]), OptTensor(saved[0])},
+                                           {dz[1], saved[1], true, OptTensor(m[1]), OptTensor(saved[2])},
+                                           {g, saved[3], true, OptTensor(g_max), OptTensor(saved[4])},
+                                           {g, x, false, OptTensor(g_max), OptTensor(saved[0])}}, rows)) {
             params.push_back(dW);
-            if (bias) params.push_back(*db);
-        };
-        of(dz[0], x, m[0], saved[0], true);
-        of(dz[1], saved[1], m[1], saved[2], true);
-        of(g, saved[3], g_max, saved[4], true);
-        of(g, x, g_max, saved[0], false);
+            if (db.has_value()) params.push_back(*db);
+        }
     }
     return {g_x, params};
 }

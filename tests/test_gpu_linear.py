@@ -1,5 +1,6 @@
 """MFMA tensor_linear against the oracle (plain matmul): rel 1e-5 / abs 1e-6 against the float64 evaluation, widened
 only by twice the distance of the float32 evaluation of the same formula from it (tests/parity.py)."""
+import ctypes
 import importlib
 
 import pytest
@@ -593,6 +594,50 @@ def test_wgrad_slices_and_tiles_over_the_chip(ops, rows, dim_in, dim_out):
     assert float((dW.double() - ref).norm()) <= 1e-6 * float(ref.norm())
     assert float((db.double() - dy.double().sum(0)).abs().max()) <= 2.0 ** -24 * rows ** 0.5 * 64
     assert torch.equal(ops.tensor_linear_wgrad(0, dy, x), dW)
+
+
+class _WgradJob(ctypes.Structure):
+    _fields_ = [("dy", ctypes.c_void_p), ("x", ctypes.c_void_p), ("dy_bound", ctypes.c_void_p), ("n_dy_bound", ctypes.c_long),
+                ("x_bound", ctypes.c_void_p), ("n_x_bound", ctypes.c_long), ("bias_rows", ctypes.c_long), ("dim_in", ctypes.c_int),
+                ("dim_out", ctypes.c_int), ("dW", ctypes.c_void_p), ("db", ctypes.c_void_p)]
+
+
+@pytest.mark.parametrize("rows,dims", [(4096, [(4, 4)]), (4097, [(128, 132), (256, 128), (4, 300)]), (20011, [(64, 64)] * 6),
+                                       (5000, [(1024, 640), (1024, 1024), (512, 512)]), (40003, [(128, 256), (256, 256), (256, 256), (128, 256)])])
+def test_weight_gradients_of_several_layers_in_one_launch(ops, rows, dims):
+    """Products that share a launch, more than one launch holds and more tiles than it takes, with and without bias, with bounds given
+    (short and long arrays, two products with one of them), from the data, biases of a part of the rows, an output off the 16-byte
+    grid: float64 as for one product, and the same products taken singly to the order of their slices."""
+    L = importlib.import_module("learned-dynamics_amd._lib")
+    lib, g = L.load(), torch.Generator(device="cuda").manual_seed(rows)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    jobs, held = (_WgradJob * len(dims))(), []
+    shared = torch.randn(rows, max(k for k, _ in dims), device="cuda", generator=g)
+    for k, (dim_in, dim_out) in enumerate(dims):
+        x = shared if dim_in == shared.shape[1] else torch.randn(rows, dim_in, device="cuda", generator=g)
+        dy = torch.randn(rows, dim_out, device="cuda", generator=g)
+        bounds = [None, None] if k % 3 == 2 else [dy.abs().amax(1), x.abs().amax(1)]
+        out = torch.full((dim_in * dim_out + 8,), float("nan"), device="cuda")
+        dW, db = out[k % 2:][:dim_in * dim_out], torch.full((dim_out,), float("nan"), device="cuda")
+        bias_rows = rows if k % 2 else rows // 2 + 1
+        jobs[k] = _WgradJob(dy.data_ptr(), x.data_ptr(), *(v for b in bounds for v in (None if b is None else b.data_ptr(), rows)), bias_rows,
+                            dim_in, dim_out, dW.data_ptr(), None if k == 3 else db.data_ptr())
+        held.append((x, dy, bounds, out, dW, db, bias_rows))
+    size = ctypes.c_size_t()
+    L.check(lib.mg_tensor_linear_wgrad_f16x2_many_workspace_bytes(ctypes.byref(jobs), len(dims), rows, ctypes.byref(size)))
+    ws = torch.empty(size.value, dtype=torch.uint8, device="cuda")
+    L.check(lib.mg_tensor_linear_wgrad_f16x2_many(ctypes.byref(jobs), len(dims), rows, ws.data_ptr(), stream))
+    for k, (x, dy, bounds, out, dW, db, bias_rows) in enumerate(held):
+        ref = dy.double().t() @ x.double()
+        assert float((dW.reshape(ref.shape).double() - ref).norm()) <= 1e-6 * float(ref.norm()), k
+        one = ops.tensor_linear_wgrad(0, dy, x, *(None if b is None else b[:, None] for b in bounds))
+        assert float((dW.reshape(ref.shape) - one).norm()) <= 1e-6 * float(ref.norm()), k
+        assert int(out.isnan().sum()) == 8, k
+        if k == 3:
+            assert db.isnan().all()
+        else:
+            assert float((db.double() - dy[:bias_rows].double().sum(0)).abs().max()) <= 2.0 ** -24 * rows ** 0.5 * 64, k
+    assert lib.mg_tensor_linear_wgrad_f16x2_many(ctypes.byref(jobs), len(dims), 4095, ws.data_ptr(), stream) != 0
 
 
 
