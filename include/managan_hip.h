@@ -481,6 +481,12 @@ int mg_tensor_linear_wgrad_f16x2_rows(const float* dy, const float* x, const flo
 int mg_tensor_linear_wgrad_f16x2_groups(const float* dy, const float* x, const float* dy_bound, long n_dy_bound,
                                         const float* x_rowmax, int groups, long rows, int dim_in, int dim_out, void* workspace,
                                         float* dW, mg_stream_t stream);
+/* dW of tensors of 3^inds components (as mg_tensor_linear_wgrad) with one dimension of at most 16 and the other of 64 or more: fp32, reads
+ * its operands as they lie.  The wider operand is 16-byte aligned.  db (dim_out; plain rows) unless NULL: the sums of dy's columns. */
+int mg_tensor_linear_wgrad_narrow_supported(int inds, long rows, int dim_in, int dim_out);   /* returns 0 / 1, not a status */
+int mg_tensor_linear_wgrad_narrow_workspace_bytes(long rows, int dim_in, int dim_out, size_t* bytes /* host */);
+int mg_tensor_linear_wgrad_narrow(int inds, const float* dy, const float* x, long rows, int dim_in, int dim_out, void* workspace,
+                                  float* dW, float* db, mg_stream_t stream);
 /* Several of them over the same rows, as few launches as their sizes allow (the weight gradients of an MLP's layers).  db NULL: not
  * wanted; a bound NULL: taken from the data.  workspace: mg_tensor_linear_wgrad_f16x2_many_workspace_bytes of the same jobs. */
 #define MG_WGRAD_F16X2_JOBS 4      /* products of one launch at most */

@@ -66,6 +66,9 @@ _SIGNATURES = {
     "mg_tensor_linear_wgrad_f16x2": [vp, vp, vp, i64, vp, i64, i64, i32, i32, vp, vp, vp, vp],
     "mg_tensor_linear_wgrad_f16x2_many": [vp, i32, i64, vp, vp],
     "mg_tensor_linear_wgrad_f16x2_many_workspace_bytes": [vp, i32, i64, vp],
+    "mg_tensor_linear_wgrad_narrow": [i32, vp, vp, i64, i32, i32, vp, vp, vp, vp],
+    "mg_tensor_linear_wgrad_narrow_supported": [i32, i64, i32, i32],
+    "mg_tensor_linear_wgrad_narrow_workspace_bytes": [i64, i32, i32, vp],
     "mg_tensor_linear_wgrad_f16x2_groups": [vp, vp, vp, i64, vp, i32, i64, i32, i32, vp, vp, vp],
     "mg_tensor_linear_products": [vp, i64, i32, vp, i64, i32, i32, vp, vp, vp],
     "mg_tensor_linear_rows": [vp, i64, i64, vp, i64, i64, i32, i32, i32, vp, vp],

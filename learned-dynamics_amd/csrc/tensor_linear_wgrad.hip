@@ -626,6 +626,27 @@ __global__ void __launch_bounds__(256) wgrad_reduce_kernel(const float* __restri
     }
 }
 
+// Sums of planes of few quads and many slices: 16 threads a quad, whose sums are added in their order: one
+// thread a quad took 10 to 13 us for planes of 1000 quads and 192 to 512 slices, four workgroups, of which each load is waited for.
+__device__ __forceinline__ float4 sum_of_slices(const float4* __restrict__ part, int quads, int splits, int k, float4* shared) {
+    const int z = threadIdx.x >> 4;
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto add = [&](const float4& v) { s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w; };
+    if (k < quads) {
+        int j = z;
+        for (; j + 48 < splits; j += 64) {
+            const float4 v0 = part[(long)j * quads + k], v1 = part[(long)(j + 16) * quads + k], v2 = part[(long)(j + 32) * quads + k],
+                         v3 = part[(long)(j + 48) * quads + k];
+            add(v0); add(v1); add(v2); add(v3);
+        }
+        for (; j < splits; j += 16) add(part[(long)j * quads + k]);
+    }
+    shared[threadIdx.x] = s;
+    __syncthreads();
+    s = shared[threadIdx.x & 15];
+    for (int j = 1; j < 16; j++) add(shared[16 * j + (threadIdx.x & 15)]);
+    return s;
+}
 // the same for the planes of several products: quad k of a plane goes to the segment that holds it
 struct WgradSegments {
     float* out[2 * MG_WGRAD_F16X2_JOBS];
@@ -633,11 +654,15 @@ struct WgradSegments {
     int count;
     bool aligned;                                          // every out is 16-byte aligned
 };
+template <bool MANY>
 __global__ void __launch_bounds__(256) wgrad_reduce_f16x2_kernel(const float4* __restrict__ part, int quads, int splits,
                                                                  const WgradSegments seg) {
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= quads) return;
+    __shared__ float4 shared[MANY ? 256 : 1];
+    const int k = MANY ? 16 * blockIdx.x + (threadIdx.x & 15) : 256 * blockIdx.x + threadIdx.x;
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (MANY) s = sum_of_slices(part, quads, splits, k, shared);
+    if (k >= quads || (MANY && threadIdx.x >= 16)) return;
+    if constexpr (!MANY) {
     auto add = [&](const float4& v) { s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w; };
     int z = 0;
     for (; z + 8 <= splits; z += 8) {                      // eight loads in flight, added in slice order
@@ -648,6 +673,7 @@ __global__ void __launch_bounds__(256) wgrad_reduce_f16x2_kernel(const float4* _
         for (int u = 0; u < 8; u++) add(v[u]);
     }
     for (; z < splits; z++) add(part[(long)z * quads + k]);
+    }
     float* out = seg.out[0];
     int first = 0;
 #pragma unroll
@@ -657,6 +683,141 @@ __global__ void __launch_bounds__(256) wgrad_reduce_f16x2_kernel(const float4* _
     if (seg.aligned) *reinterpret_cast<float4*>(out) = s;
     else { out[0] = s.x; out[1] = s.y; out[2] = s.z; out[3] = s.w; }
 }
+
+// ---------------------------------------------------------------------------------------- one dimension of at most 16
+// P[k, i] = sum_{r, t} narrow[r, k, t] wide[r, i, t] with k < n <= 16: two to thirty-two multiply-adds a float of the wide operand, which
+// is read once, 16 bytes a lane, in whatever layout of components it has: nothing is transposed, and products and sums are fp32, so
+// no bounds are needed either.  A lane holds the n results of four channels, L lanes a row, 256 / L rows at a time; the narrow
+// operand's rows lie in LDS, where all lanes of a row read the same words.
+// Bound by memory: 1.5 M rows 16 -> 512 at 4.5 TB/s.  Against the split-fp16 product with its padding to 128 x 128, its row maxima and,
+// for tensors, its transposed copies: that one 1242 -> 697 us, 73 728 rows 1280 -> 16 168 -> 107, 16 -> 256 52 -> 29, 8192 rows of
+// three components 1 -> 128 and 128 -> 1 42 -> 8, 128 -> 16 41 -> 18, of nine 128 -> 1 68 -> 11.
+// BIAS: the sums of the columns of dy as well (of plain rows), where dy is the wide operand or the narrow one; behind the plane (n, dim).
+constexpr int kNarrow = 16, kNarrowRows = 64;
+enum NarrowBias { kNoBias, kOfWide, kOfNarrow };
+template <int T, int N, int BIAS = kNoBias>
+__global__ void __launch_bounds__(256) wgrad_narrow_kernel(const float* __restrict__ narrow, int n, const float* __restrict__ wide,
+                                                           int dim, long R, long rows_per_block, int L, long plane,
+                                                           float* __restrict__ part) {
+    constexpr int kAhead = T == 1 ? 8 : T == 3 ? 4 : 1;       // rows requested together
+    __shared__ __attribute__((aligned(16))) float buf[kNarrowRows * N * T > 1024 ? kNarrowRows * N * T : 1024];
+    const int l = threadIdx.x & (L - 1), group = threadIdx.x / L, groups = 256 / L;
+    const int quad = blockIdx.x * L + l;
+    const bool live = quad < dim / 4;
+    const float* own = wide + (live ? quad : 0) * 4L * T;
+    const long r_lo = (long)blockIdx.y * rows_per_block, r_hi = r_lo + rows_per_block < R ? r_lo + rows_per_block : R;
+    float acc[N][4];
+#pragma unroll
+    for (int k = 0; k < N; k++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[k][j] = 0.f;
+    float column[4] = {0.f, 0.f, 0.f, 0.f};                   // of the wide operand; of the narrow one in column[0], its column ...
+    const int own_k = threadIdx.x & (kNarrow - 1), own_rows = threadIdx.x / kNarrow;      // ... and rows of this thread
+    for (long r = r_lo; r < r_hi; r += kNarrowRows) {
+        const int rows = r_hi - r < kNarrowRows ? (int)(r_hi - r) : kNarrowRows;
+        __syncthreads();
+        // (what lies between n and N is never used)
+        for (int at = threadIdx.x; at < rows * n * T; at += 256) {
+            const int row = at / (n * T);
+            buf[row * (N * T) + (at - row * (n * T))] = narrow[r * n * T + at];
+        }
+        __syncthreads();
+        if (BIAS == kOfNarrow && blockIdx.x == 0 && own_k < n)
+            for (int row = own_rows; row < rows; row += 256 / kNarrow) column[0] += buf[row * N + own_k];
+        for (int first = group; first < rows; first += kAhead * groups) {
+            union { float4 v[T]; float f[4 * T]; } x[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) {
+                const int row = first + u * groups < rows ? first + u * groups : rows - 1;
+                const float4* from = reinterpret_cast<const float4*>(own + (r + row) * ((long)dim * T));
+#pragma unroll
+                for (int t = 0; t < T; t++) x[u].v[t] = from[t];
+            }
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) {
+                const int row = first + u * groups;
+                if (row < rows) {
+                    const float* b = buf + row * (N * T);
+#pragma unroll
+                    for (int k = 0; k < N; k++)
+#pragma unroll
+                        for (int t = 0; t < T; t++)
+#pragma unroll
+                            for (int j = 0; j < 4; j++) acc[k][j] = fmaf(b[k * T + t], x[u].f[j * T + t], acc[k][j]);
+                    if constexpr (BIAS == kOfWide)
+#pragma unroll
+                        for (int j = 0; j < 4; j++) column[j] += x[u].f[j];
+                }
+            }
+        }
+    }
+    // the groups' sums, added in their order
+    float4* sums = reinterpret_cast<float4*>(buf);
+    auto combine = [&](int k, const float (&own_sum)[4]) {
+        __syncthreads();
+        sums[threadIdx.x] = make_float4(own_sum[0], own_sum[1], own_sum[2], own_sum[3]);
+        __syncthreads();
+        if (group == 0 && live) {
+            float4 s = sums[l];
+            for (int g = 1; g < groups; g++) {
+                const float4 v = sums[g * L + l];
+                s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+            }
+            *reinterpret_cast<float4*>(part + blockIdx.y * plane + (long)k * dim + 4 * quad) = s;
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < N; k++)
+        if (k < n) combine(k, acc[k]);                        // (uniform)
+    if constexpr (BIAS == kOfWide) combine(n, column);
+    if (BIAS == kOfNarrow && blockIdx.x == 0) {
+        __syncthreads();
+        buf[threadIdx.x] = column[0];
+        __syncthreads();
+        if (threadIdx.x < kNarrow) {
+            float s = buf[threadIdx.x];
+            for (int j = 1; j < 256 / kNarrow; j++) s += buf[kNarrow * j + threadIdx.x];
+            part[blockIdx.y * plane + (long)n * dim + threadIdx.x] = s;
+        }
+    }
+}
+
+// quad q of the plane (n, dim) to dW, transposed where x is the narrow operand, and those behind it to db (n_bias floats)
+__global__ void __launch_bounds__(256) wgrad_narrow_reduce_kernel(const float4* __restrict__ part, int quads, int splits, int dim,
+                                                                  int n, bool transposed, int n_bias, float* __restrict__ dW,
+                                                                  float* __restrict__ db) {
+    __shared__ float4 shared[256];
+    const int q = 16 * blockIdx.x + (threadIdx.x & 15);
+    const float4 s = sum_of_slices(part, quads, splits, q, shared);
+    if (threadIdx.x >= 16 || q >= quads) return;
+    const float v[4] = {s.x, s.y, s.z, s.w};
+    const int k = q / (dim / 4), i = 4 * (q - k * (dim / 4));
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if (k < n) dW[transposed ? (long)(i + j) * n + k : (long)k * dim + i + j] = v[j];
+        else if (i + j < n_bias) db[i + j] = v[j];
+    }
+}
+
+// lanes of a row, channel blocks, rows of a workgroup and their number: about four workgroups on each compute unit, of 64 rows at least
+struct NarrowPlan {
+    int lanes, blocks, n, dim;
+    long rows, splits, plane;
+};
+NarrowPlan narrow_plan(long R, int dim_in, int dim_out) {
+    NarrowPlan p;
+    p.n = dim_in < dim_out ? dim_in : dim_out;
+    p.dim = dim_in < dim_out ? dim_out : dim_in;
+    p.lanes = 16;
+    while (p.lanes < 64 && 4 * p.lanes < p.dim) p.lanes *= 2;
+    p.blocks = (int)ceil_div(p.dim, 4 * p.lanes);
+    const long most = ceil_div(R, kNarrowRows), want = ceil_div(1024, p.blocks), s = want < most ? want : most;
+    p.rows = ceil_div(ceil_div(R, s < 1 ? 1 : s), kNarrowRows) * kNarrowRows;
+    p.splits = ceil_div(R, p.rows);
+    p.plane = (long)p.n * p.dim;
+    return p;
+}
+long narrow_bias_floats(int dim_in, int dim_out) { return dim_in < dim_out ? dim_out : kNarrow; }
 
 // rows per slice and number of slices for a problem (the same on the sizing and the launching side)
 // resident_groups = 0: aim at ~4 workgroups per CU; otherwise the number of workgroups the chip holds at once, which
@@ -801,7 +962,9 @@ static int wgrad_f16x2(const mg_wgrad_f16x2* jobs, int count, int x_groups, long
     MG_REQUIRE(items < (1L << 31) - 8 && plane / 4 < (1L << 31), "mg_tensor_linear_wgrad_f16x2: grid too large");
     hipLaunchKernelGGL(wgrad_f16x2_kernel, dim3((unsigned)(8 * ceil_div(items, 8))), dim3(256), 0, st, all);
     const int quads = (int)(plane / 4);
-    hipLaunchKernelGGL(wgrad_reduce_f16x2_kernel, dim3((unsigned)ceil_div(quads, 256)), dim3(256), 0, st,
+    const bool many = splits > 32;
+    hipLaunchKernelGGL(many ? wgrad_reduce_f16x2_kernel<true> : wgrad_reduce_f16x2_kernel<false>,
+                       dim3((unsigned)ceil_div(quads, many ? 16 : 256)), dim3(256), 0, st,
                        reinterpret_cast<const float4*>(all.parts), quads, (int)splits, seg);
     return check_launch("mg_tensor_linear_wgrad_f16x2");
 }
@@ -874,6 +1037,54 @@ int mg_tensor_linear_wgrad_f16x2(const float* dy, const float* x, const float* d
                                  void* workspace, float* dW, float* db, mg_stream_t stream) {
     return mg_tensor_linear_wgrad_f16x2_rows(dy, x, dy_bound, n_dy_bound, x_bound, n_x_bound, rows, rows, dim_in, dim_out,
                                              workspace, dW, db, stream);
+}
+
+int mg_tensor_linear_wgrad_narrow_supported(int inds, long rows, int dim_in, int dim_out) {
+    const int n = dim_in < dim_out ? dim_in : dim_out, dim = dim_in < dim_out ? dim_out : dim_in, T = inds == 0 ? 1 : inds == 1 ? 3 : 9;
+    return inds >= 0 && inds <= 2 && rows >= 1 && rows < (1L << 31) && n >= 1 && n <= kNarrow && n * T <= 3 * kNarrow && dim % 4 == 0 &&
+           dim >= 64 && dim >= 4 * n && dim <= 65536;
+}
+
+int mg_tensor_linear_wgrad_narrow_workspace_bytes(long rows, int dim_in, int dim_out, size_t* bytes) {
+    MG_REQUIRE(bytes != nullptr && rows >= 0 && dim_in >= 1 && dim_out >= 1, "mg_tensor_linear_wgrad_narrow_workspace_bytes: bad argument");
+    const NarrowPlan p = narrow_plan(rows > 0 ? rows : 1, dim_in, dim_out);
+    *bytes = (size_t)p.splits * (p.plane + narrow_bias_floats(dim_in, dim_out)) * sizeof(float) + 16;
+    return MG_OK;
+}
+
+int mg_tensor_linear_wgrad_narrow(int inds, const float* dy, const float* x, long rows, int dim_in, int dim_out, void* workspace,
+                                  float* dW, float* db, mg_stream_t stream) {
+    MG_REQUIRE(mg_tensor_linear_wgrad_narrow_supported(inds, rows, dim_in, dim_out),
+               "mg_tensor_linear_wgrad_narrow: one dimension of at most 16 (5 in rank 2), the other of 64 or more, in fours");
+    const bool of_x = dim_in < dim_out;                       // x is the narrow operand
+    const float *narrow = of_x ? x : dy, *wide = of_x ? dy : x;
+    MG_REQUIRE(dy && x && workspace && dW && aligned16(wide), "mg_tensor_linear_wgrad_narrow: null or unaligned pointer");
+    hipStream_t st = (hipStream_t)stream;
+    MG_REQUIRE(inds == 0 || db == nullptr, "mg_tensor_linear_wgrad_narrow: the bias gradient is defined for plain rows only");
+    NarrowPlan p = narrow_plan(rows, dim_in, dim_out);
+    if (db) p.plane += narrow_bias_floats(dim_in, dim_out);
+    float* part = reinterpret_cast<float*>((reinterpret_cast<uintptr_t>(workspace) + 15) & ~uintptr_t(15));
+    const dim3 grid((unsigned)p.blocks, (unsigned)p.splits);
+    const auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, narrow, p.n, wide, p.dim, rows, p.rows, p.lanes, p.plane, part);
+    };
+    const auto of_width = [&](auto width) {
+        constexpr int N = decltype(width)::value;
+        if (inds == 0 && db) run(of_x ? wgrad_narrow_kernel<1, N, kOfWide> : wgrad_narrow_kernel<1, N, kOfNarrow>);
+        else if (inds == 0) run(wgrad_narrow_kernel<1, N>);
+        else if (inds == 1) run(wgrad_narrow_kernel<3, N>);
+        else if constexpr (N <= 5) run(wgrad_narrow_kernel<9, N>);
+    };
+    if (p.n <= 1) of_width(std::integral_constant<int, 1>{});
+    else if (p.n <= 2) of_width(std::integral_constant<int, 2>{});
+    else if (p.n <= 4) of_width(std::integral_constant<int, 4>{});
+    else if (p.n == 5) of_width(std::integral_constant<int, 5>{});
+    else if (p.n <= 8) of_width(std::integral_constant<int, 8>{});
+    else of_width(std::integral_constant<int, kNarrow>{});
+    const int quads = (int)(p.plane / 4);
+    hipLaunchKernelGGL(wgrad_narrow_reduce_kernel, dim3((unsigned)ceil_div(quads, 16)), dim3(256), 0, st,
+                       reinterpret_cast<const float4*>(part), quads, (int)p.splits, p.dim, p.n, of_x, dim_out, dW, db);
+    return check_launch("mg_tensor_linear_wgrad_narrow");
 }
 
 int mg_tensor_linear_wgrad(int inds, const float* dy, const float* x, long rows, int dim_in, int dim_out,

@@ -414,6 +414,21 @@ std::tuple<at::Tensor, OptTensor> linear_fwd(int64_t inds, const at::Tensor& W, 
     return {y, ymax.defined() ? OptTensor(ymax) : OptTensor()};
 }
 
+// Weight gradients with one dimension of at most 16 from where the split-fp16 products take them (below, fp32 products in the order
+// of the rows): fp32, the wide operand read once, at half their time or less (figures at the kernel).
+bool narrow_wgrad_takes(int64_t inds, int64_t rows, const at::Tensor& dy, const at::Tensor& x, int64_t dim_in, int64_t dim_out) {
+    return mg_get_linear_mode() == kModeF16x2 && rows * (inds == 0 ? 1 : inds == 1 ? 3 : 9) >= 4096 &&
+           mg_tensor_linear_wgrad_narrow_supported((int)inds, rows, (int)dim_in, (int)dim_out) && aligned16(dim_in < dim_out ? dy : x);
+}
+void narrow_wgrad(int64_t inds, int64_t rows, const at::Tensor& dy, const at::Tensor& x, int64_t dim_in, int64_t dim_out, at::Tensor& dW,
+                  float* db = nullptr) {
+    size_t n = 0;
+    check(mg_tensor_linear_wgrad_narrow_workspace_bytes(rows, (int)dim_in, (int)dim_out, &n));
+    at::Tensor ws = bytes_like(x, n);
+    check(mg_tensor_linear_wgrad_narrow((int)inds, fp(dy), fp(x), rows, (int)dim_in, (int)dim_out, ws.data_ptr(), fp(dW), db,
+                                        stream_of(x)));
+}
+
 // dW (and with want_bias db): see ops.tensor_linear_wgrad
 std::tuple<at::Tensor, OptTensor> linear_wgrad(int64_t inds, const at::Tensor& dy, const at::Tensor& x,
                                                const OptTensor& dy_bound, const OptTensor& x_bound, bool want_bias) {
@@ -434,7 +449,12 @@ std::tuple<at::Tensor, OptTensor> linear_wgrad(int64_t inds, const at::Tensor& d
         return bytes_like(x, n);
     };
     OptTensor db;
-    if (inds == 0 && mode == kModeF16x2 && aligned16(x) && aligned16(dy) &&
+    if (narrow_wgrad_takes(inds, rows, dy, x, dim_in, dim_out)) {
+        at::Tensor bias_grad;
+        if (want_bias) bias_grad = floats(x, {dim_out});
+        narrow_wgrad(inds, rows, dy, x, dim_in, dim_out, dW, want_bias ? fp(bias_grad) : nullptr);
+        if (want_bias) db = bias_grad;
+    } else if (inds == 0 && mode == kModeF16x2 && aligned16(x) && aligned16(dy) &&
         mg_tensor_linear_wgrad_f16x2_supported(rows, (int)dim_in, (int)dim_out)) {
         if (dy_bound.has_value()) check_input(*dy_bound, "dy_bound");
         if (x_bound.has_value()) check_input(*x_bound, "x_bound");
@@ -937,8 +957,9 @@ std::tuple<OptTensor, Tensors> row_linears_bwd(const at::Tensor& dy, const at::T
     const bool split_x = f16x2 && f16x2_takes(R, O, G * C, dy) && (T == 1 || component_rows_take(R, O, C, false));
     const bool split_W = f16x2 && aligned16(x) && aligned16(dy) && (T == 1 || std::max(C, O) <= 256) &&
                          mg_tensor_linear_wgrad_f16x2_supported(R, (int)C, (int)O);
+    const bool narrow = narrow_wgrad_takes(0, R, dy, x, G * C, O);
     OptTensor dx, dy_max;
-    if ((want_x && split_x) || (want_W && split_W)) dy_max = row_absmax(dy);
+    if ((want_x && split_x) || (want_W && split_W && !narrow)) dy_max = row_absmax(dy);
     if (want_x) {
         // (one linear: the columns' scales are those of the transposed weights' rows, one for each channel of each x_k)
         const at::Tensor Wt = (G == 1 ? W[0] : at::cat(W, 1)).t();
@@ -951,9 +972,11 @@ std::tuple<OptTensor, Tensors> row_linears_bwd(const at::Tensor& dy, const at::T
     if (want_W) {
         at::Tensor all = floats(x, {O, G * C});
         size_t n = 0;
-        check(mg_tensor_linear_wgrad_workspace_bytes(R, (int)(G * C), (int)O, &n));
+        if (!narrow) check(mg_tensor_linear_wgrad_workspace_bytes(R, (int)(G * C), (int)O, &n));
         at::Tensor ws = bytes_like(x, n);
-        if (split_W) {
+        if (narrow) {
+            narrow_wgrad(0, R, dy, x, G * C, O, all);
+        } else if (split_W) {
             if (!x_max.has_value()) x_max = row_absmax(x.view({R * G, C}));
             check(mg_tensor_linear_wgrad_f16x2_groups(fp(dy), fp(x), fp(dy_max), R, fp(x_max), (int)G, R, (int)(G * C), (int)O,
                                                       ws.data_ptr(), fp(all), stream_of(x)));

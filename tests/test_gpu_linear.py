@@ -596,6 +596,32 @@ def test_wgrad_slices_and_tiles_over_the_chip(ops, rows, dim_in, dim_out):
     assert torch.equal(ops.tensor_linear_wgrad(0, dy, x), dW)
 
 
+@pytest.mark.parametrize("inds,rows,dims", [(0, 4096, (64, 1)), (0, 4097, (16, 260)), (0, 70001, (1280, 13)), (0, 5000, (3, 64)),
+                                            (1, 1366, (1, 128)), (1, 9001, (128, 16)), (1, 3000, (76, 5)), (2, 456, (64, 1)),
+                                            (2, 2001, (4, 100)), (2, 2001, (300, 5))])
+def test_weight_gradient_with_one_narrow_dimension(ops, inds, rows, dims):
+    """One dimension of at most 16: lanes without channels, slices and chunks cut short, every width the kernel is compiled for and both
+    operands narrow.  float32 products and sums of few rows each: 2^-24 a product and addition, in the 2-norm; rows with infinities
+    reach the entries that they reach in the formula and no others."""
+    lib = importlib.import_module("learned-dynamics_amd._lib").load()
+    dim_in, dim_out = dims
+    assert lib.mg_tensor_linear_wgrad_narrow_supported(inds, rows, dim_in, dim_out)
+    g, T = torch.Generator().manual_seed(rows), 3 ** inds
+    dy, x = (torch.randn(rows, d, *[3] * inds, generator=g).cuda() for d in (dim_out, dim_in))
+    plain = lambda t: t.double().reshape(rows, -1, T).transpose(1, 2).reshape(rows * T, -1)
+    dW = ops.tensor_linear_wgrad(inds, dy, x)
+    ref = plain(dy).t() @ plain(x)
+    assert float((dW.double() - ref).norm()) <= 4e-7 * float(ref.norm())
+    assert torch.equal(ops.tensor_linear_wgrad(inds, dy, x), dW)
+    if inds == 0:
+        with_bias, db = ops.tensor_linear_wgrad(0, dy, x, want_bias=True)
+        assert torch.equal(with_bias, dW)
+        assert float((db.double() - dy.double().sum(0)).abs().max()) <= 2.0 ** -24 * rows ** 0.5 * 64
+    dy[-1, 0] = float("inf")
+    marked = ops.tensor_linear_wgrad(inds, dy, x)
+    assert not marked[0].isfinite().any() and torch.equal(marked[1:], dW[1:])
+
+
 class _WgradJob(ctypes.Structure):
     _fields_ = [("dy", ctypes.c_void_p), ("x", ctypes.c_void_p), ("dy_bound", ctypes.c_void_p), ("n_dy_bound", ctypes.c_long),
                 ("x_bound", ctypes.c_void_p), ("n_x_bound", ctypes.c_long), ("bias_rows", ctypes.c_long), ("dim_in", ctypes.c_int),
