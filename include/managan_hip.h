@@ -439,6 +439,9 @@ typedef struct mg_mlp_leaky_f16x2_grad {
 int mg_mlp_leaky_f16x2_supported(int dim_in, int dim, int dim_out);      /* returns 0 / 1, not a status */
 int mg_mlp_leaky_f16x2_forward(const mg_mlp_leaky_f16x2* args /* host */, mg_stream_t stream);
 int mg_mlp_leaky_f16x2_adjoint(const mg_mlp_leaky_f16x2_grad* args /* host */, mg_stream_t stream);
+/* the same of x + y: x is added to y, dy to dx (dim_in == dim_out) */
+int mg_mlp_leaky_f16x2_residual_forward(const mg_mlp_leaky_f16x2* args /* host */, mg_stream_t stream);
+int mg_mlp_leaky_f16x2_residual_adjoint(const mg_mlp_leaky_f16x2_grad* args /* host */, mg_stream_t stream);
 /* The nonlinear layers of an MLP whose result is only needed summed over the rows of segments (archs/diffuser_atoms15.py:98-110
  * under edges_reduce_src, :244-246): out[s] = sum over the rows r of segment s of f(W2 f(W1 x[r] + b1) + b2), f = LeakyReLU(0.1),
  * x (rows, dim_in), both layers `dim` wide, out (n_out, dim).  Rows are sorted by segment (seg ascending, row_ptr its CSR form);

@@ -151,6 +151,8 @@ _SIGNATURES = {
     "mg_mlp_leaky_f16x2_supported": [i32, i32, i32],
     "mg_mlp_leaky_f16x2_forward": [vp, vp],
     "mg_mlp_leaky_f16x2_adjoint": [vp, vp],
+    "mg_mlp_leaky_f16x2_residual_forward": [vp, vp],
+    "mg_mlp_leaky_f16x2_residual_adjoint": [vp, vp],
     "mg_mlp_leaky_rowsum_f16x2_workspace_bytes": [i64, i32, ctypes.POINTER(ctypes.c_size_t)],
     "mg_mlp_leaky_rowsum_f16x2": [vp, vp, vp, vp, vp, i64, i32, i32, vp, vp, i64, vp, vp, vp],
     "mg_silu_rows_fwd": [vp, i64, i32, i32, vp, vp, vp],

@@ -223,8 +223,7 @@ class MLP(nn.Module):
         """Returns mlp(x), or x + mlp(x) with plus_identity=True.  bound: upper bounds of the row
         maxima of |x| ((rows, 1) or (1, 1)) if the caller has them."""
         if diff.wants_grad(self, x):
-            y = diff.mlp_leaky(self, x)
-            return x + y if plus_identity else y
+            return diff.mlp_leaky(self, x, plus_identity)
         lead = x.shape[:-1]
         x2 = x.reshape(-1, x.shape[-1]).contiguous()
         Wd = self.lin_direct.weight

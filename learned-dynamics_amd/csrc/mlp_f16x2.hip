@@ -41,6 +41,9 @@ struct MlpArgs {
     const float* z_in[2];          // adjoint: the hidden layers' inputs of their activation, in the order they are met
     float *z[2], *h[2], *h_max[2]; // training: kept for the adjoint; adjoint: h, h_max are the gradients of z and their row maxima
     float* x_max;
+    // LEAKY: x is added to the result (K == N).  127 456 rows, 256 -> 512 -> 256: 10 us forward and 20 in the adjoint (590, 738) for
+    // the rows that the workgroup read before, where an addition of its own took 57.
+    bool residual;
 };
 
 // lanes 16 .. 31 (48 .. 63) of a and lanes 0 .. 15 (32 .. 47) of b change places; done twice, all is as before
@@ -321,12 +324,14 @@ __device__ __forceinline__ void mlp_rows(const MlpArgs& a, long tile, int widest
             for (int mi = 0; mi < MI; mi++) {
                 if (!live(mi)) continue;
                 float* out = a.y + row_of(mi, m) * N + 32 * nb + 4 * G;
+                const float* res = LEAKY && a.residual ? a.x + row_of(mi, m) * N + 32 * nb + 4 * G : nullptr;
                 const float* bias = MODE == kAdjoint ? nullptr : a.bias[2];
                 if (odd[mi]) {
 #pragma unroll 1
                     for (int q = 0; q < 16; q++) {
                         const int c = 8 * (q / 4) + q % 4, n = 32 * nb + 4 * G + c;
-                        out[c] = lds_row_in_fp32(xh + mi * 32 * O, x_lo, m, a.planes[2], w_lo, n, O, inv[n]) + (bias ? bias[n] : 0.f);
+                        out[c] = lds_row_in_fp32(xh + mi * 32 * O, x_lo, m, a.planes[2], w_lo, n, O, inv[n]) + (bias ? bias[n] : 0.f) +
+                                 (res ? res[c] : 0.f);
                     }
                     continue;
                 }
@@ -335,6 +340,10 @@ __device__ __forceinline__ void mlp_rows(const MlpArgs& a, long tile, int widest
                     const float4 iw = *reinterpret_cast<const float4*>(inv + 32 * nb + 8 * t + 4 * G);
                     float4 b = make_float4(0.f, 0.f, 0.f, 0.f);
                     if (bias) b = *reinterpret_cast<const float4*>(bias + 32 * nb + 8 * t + 4 * G);
+                    if (res) {
+                        const float4 r = *reinterpret_cast<const float4*>(res + 8 * t);
+                        b.x += r.x; b.y += r.y; b.z += r.z; b.w += r.w;
+                    }
                     *reinterpret_cast<float4*>(out + 8 * t) =
                         make_float4(acc[mi][0][4 * t] * isx[mi] * iw.x + b.x, acc[mi][0][4 * t + 1] * isx[mi] * iw.y + b.y,
                                     acc[mi][0][4 * t + 2] * isx[mi] * iw.z + b.z, acc[mi][0][4 * t + 3] * isx[mi] * iw.w + b.w);
@@ -720,11 +729,13 @@ int mg_mlp_leaky_f16x2_supported(int dim_in, int dim, int dim_out) {
     return mg_mlp_f16x2_supported(dim_in, dim) && mg_mlp_f16x2_supported(dim_out, dim);
 }
 
-int mg_mlp_leaky_f16x2_forward(const mg_mlp_leaky_f16x2* p, mg_stream_t stream) {
+static int mlp_leaky_forward(const mg_mlp_leaky_f16x2* p, bool residual, mg_stream_t stream) {
     MG_REQUIRE(p != nullptr && p->rows >= 0 && mg_mlp_leaky_f16x2_supported(p->dim_in, p->dim, p->dim_out),
                "mg_mlp_leaky_f16x2_forward: dimensions must be multiples of 32 up to %d", kMaxDim);
+    MG_REQUIRE(!residual || p->dim_in == p->dim_out, "mg_mlp_leaky_f16x2_residual_forward: dim_in == dim_out expected");
     if (p->rows == 0) return MG_OK;
     MlpArgs a{};
+    a.residual = residual;
     a.x = p->x;
     a.R = p->rows;
     a.K = p->dim_in;
@@ -745,11 +756,13 @@ int mg_mlp_leaky_f16x2_forward(const mg_mlp_leaky_f16x2* p, mg_stream_t stream) 
     return launch_leaky<kTrain>(a, (hipStream_t)stream);
 }
 
-int mg_mlp_leaky_f16x2_adjoint(const mg_mlp_leaky_f16x2_grad* p, mg_stream_t stream) {
+static int mlp_leaky_adjoint(const mg_mlp_leaky_f16x2_grad* p, bool residual, mg_stream_t stream) {
     MG_REQUIRE(p != nullptr && p->rows >= 0 && mg_mlp_leaky_f16x2_supported(p->dim_in, p->dim, p->dim_out),
                "mg_mlp_leaky_f16x2_adjoint: dimensions must be multiples of 32 up to %d", kMaxDim);
+    MG_REQUIRE(!residual || p->dim_in == p->dim_out, "mg_mlp_leaky_f16x2_residual_adjoint: dim_in == dim_out expected");
     if (p->rows == 0) return MG_OK;
     MlpArgs a{};
+    a.residual = residual;
     a.x = p->dy;
     a.R = p->rows;
     a.K = p->dim_out;
@@ -769,6 +782,11 @@ int mg_mlp_leaky_f16x2_adjoint(const mg_mlp_leaky_f16x2_grad* p, mg_stream_t str
                "mg_mlp_leaky_f16x2_adjoint: null or unaligned pointer");
     return launch_leaky<kAdjoint>(a, (hipStream_t)stream);
 }
+
+int mg_mlp_leaky_f16x2_forward(const mg_mlp_leaky_f16x2* p, mg_stream_t stream) { return mlp_leaky_forward(p, false, stream); }
+int mg_mlp_leaky_f16x2_adjoint(const mg_mlp_leaky_f16x2_grad* p, mg_stream_t stream) { return mlp_leaky_adjoint(p, false, stream); }
+int mg_mlp_leaky_f16x2_residual_forward(const mg_mlp_leaky_f16x2* p, mg_stream_t stream) { return mlp_leaky_forward(p, true, stream); }
+int mg_mlp_leaky_f16x2_residual_adjoint(const mg_mlp_leaky_f16x2_grad* p, mg_stream_t stream) { return mlp_leaky_adjoint(p, true, stream); }
 
 int mg_mlp_leaky_rowsum_f16x2_workspace_bytes(long rows, int dim, size_t* bytes) {
     MG_REQUIRE(bytes != nullptr && rows >= 0 && dim >= 0, "mg_mlp_leaky_rowsum_f16x2_workspace_bytes: bad argument");

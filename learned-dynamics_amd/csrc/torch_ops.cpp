@@ -1233,7 +1233,8 @@ bool mlp_leaky_takes(const at::Tensor& x, const Tensors& W, const Tensors& b) {
 }
 
 // saved: row maxima of |x|, then h and its row maxima of either hidden layer
-std::tuple<at::Tensor, Tensors> mlp_leaky_fwd(const at::Tensor& x, const Tensors& W, const Tensors& b) {
+// residual: of x + y
+std::tuple<at::Tensor, Tensors> mlp_leaky_fwd(const at::Tensor& x, const Tensors& W, const Tensors& b, bool residual) {
     TORCH_CHECK(mlp_leaky_takes(x, W, b), "mlp_leaky_fwd: sizes or types");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     pack_ahead({W[0], W[1], W[2], W[3], W[0].t(), W[1].t(), W[2].t(), W[3].t()});
@@ -1258,13 +1259,13 @@ std::tuple<at::Tensor, Tensors> mlp_leaky_fwd(const at::Tensor& x, const Tensors
     a.dim = (int)dim;
     a.dim_out = (int)W[2].size(0);
     a.y = fp(y);
-    check(mg_mlp_leaky_f16x2_forward(&a, stream_of(x)));
+    check((residual ? mg_mlp_leaky_f16x2_residual_forward : mg_mlp_leaky_f16x2_forward)(&a, stream_of(x)));
     run_f16x2(W[3], W[3].size(1), fp(x), rows, Bound{OptTensor(saved[0])}, OptTensor(), kActNone, true, 1, y, nullptr, true);
     return {y, saved};
 }
 
 std::tuple<OptTensor, Tensors> mlp_leaky_bwd(const at::Tensor& g, const at::Tensor& x, const Tensors& W, const Tensors& saved,
-                                             bool want_x, bool want_params) {
+                                             bool want_x, bool want_params, bool residual) {
     check_input(g, "gradient");
     TORCH_CHECK(W.size() == 4 && saved.size() == 5 && g.dim() == 2 && g.size(0) == x.size(0) && g.size(1) == W[2].size(0) && aligned16(g),
                 "mlp_leaky_bwd: sizes");
@@ -1294,7 +1295,7 @@ std::tuple<OptTensor, Tensors> mlp_leaky_bwd(const at::Tensor& g, const at::Tens
     a.dim_in = (int)W[0].size(1);
     a.dim = (int)dim;
     a.dim_out = (int)W[2].size(0);
-    check(mg_mlp_leaky_f16x2_adjoint(&a, stream_of(x)));
+    check((residual ? mg_mlp_leaky_f16x2_residual_adjoint : mg_mlp_leaky_f16x2_adjoint)(&a, stream_of(x)));
     if (want_x) run_f16x2(W[3].t(), W[3].size(0), fp(g), rows, Bound{OptTensor(g_max)}, OptTensor(), kActNone, true, 1, *g_x, nullptr, false);
     Tensors params;
     if (want_params) {
@@ -1718,8 +1719,9 @@ void register_ops(pybind11::module_& m) {
     m.def("mlp_silu_fwd", &mlp_silu_fwd);
     m.def("mlp_silu_bwd", &mlp_silu_bwd);
     m.def("mlp_leaky_takes", &mlp_leaky_takes);
-    m.def("mlp_leaky_fwd", &mlp_leaky_fwd);
-    m.def("mlp_leaky_bwd", &mlp_leaky_bwd);
+    m.def("mlp_leaky_fwd", &mlp_leaky_fwd, py::arg("x"), py::arg("W"), py::arg("b"), py::arg("residual") = false);
+    m.def("mlp_leaky_bwd", &mlp_leaky_bwd, py::arg("g"), py::arg("x"), py::arg("W"), py::arg("saved"), py::arg("want_x"),
+          py::arg("want_params"), py::arg("residual") = false);
     m.def("edge_encode_fwd", &edge_encode_fwd);
     m.def("edge_encode_bwd", &edge_encode_bwd);
     m.def("combine_dual_fwd", &combine_dual_fwd);

@@ -314,11 +314,12 @@ def _mlp_silu_pair(mlp, x):
 
 class _MlpLeaky(torch.autograd.Function):
     """bee_layers.MLP on rows: the layers as one kernel each way, the direct map added to their result.  params: weight and bias of
-    the three layers, then the direct map's weight."""
+    the three layers, then the direct map's weight.  residual: of x + y, added where the kernels write y and the gradient of x."""
 
     @staticmethod
-    def forward(ctx, x, *params):
-        y, rows = ops.mlp_leaky_fwd(x, params[0:6:2] + params[6:], params[1:6:2])
+    def forward(ctx, residual, x, *params):
+        ctx.residual = residual
+        y, rows = ops.mlp_leaky_fwd(x, params[0:6:2] + params[6:], params[1:6:2], residual)
         ctx.save_for_backward(x, *params, *(rows if any(ctx.needs_input_grad) else ()))
         ctx.set_materialize_grads(False)
         return y
@@ -327,17 +328,18 @@ class _MlpLeaky(torch.autograd.Function):
     def backward(ctx, g):
         x, *saved = ctx.saved_tensors
         params, rows = saved[:7], saved[7:]
-        need = ctx.needs_input_grad
+        need, residual = ctx.needs_input_grad[1:], ctx.residual
         if g is None:
-            return (None,) * len(need)
-        pieces = _gradients_in_pieces(lambda x, *p: (_mlp_leaky_rows(p, x),), (x, *params), need, (g,))
+            return (None,) * (1 + len(need))
+        pieces = _gradients_in_pieces(lambda x, *p: (x + _mlp_leaky_rows(p, x) if residual else _mlp_leaky_rows(p, x),), (x, *params),
+                                      need, (g,))
         if pieces is not None:
-            return pieces
+            return (None, *pieces)
         g = g.contiguous()
         if g.data_ptr() % 16:
             g = g.clone()
-        g_x, d_params = ops.mlp_leaky_bwd(g, x, params[0:6:2] + params[6:], rows, need[0], any(need[1:]))
-        return (g_x if need[0] else None,) + tuple(d if nd else None for d, nd in zip(d_params or [None] * 7, need[1:]))
+        g_x, d_params = ops.mlp_leaky_bwd(g, x, params[0:6:2] + params[6:], rows, need[0], any(need[1:]), residual)
+        return (None, g_x if need[0] else None) + tuple(d if nd else None for d, nd in zip(d_params or [None] * 7, need[1:]))
 
 
 def _mlp_leaky_rows(params, x):
@@ -348,17 +350,21 @@ def _mlp_leaky_rows(params, x):
     return tensor_linear(0, Wd, x, sequential=True) + tensor_linear(0, W2, F.leaky_relu(z, 0.1), bias=b2, x_bound=b, sequential=True)
 
 
-def mlp_leaky(mlp, x):
-    """bee_layers.MLP: lin_direct(x) + layers(x) with LeakyReLU(0.1) (archs/diffuser_atoms15.py:98-110)."""
+def mlp_leaky(mlp, x, residual=False):
+    """bee_layers.MLP: lin_direct(x) + layers(x) with LeakyReLU(0.1) (archs/diffuser_atoms15.py:98-110); x + that with residual."""
     params = [*_mlp_parameters(mlp), mlp.lin_direct.weight]
-    lead, x = x.shape[:-1], x.reshape(-1, x.shape[-1]).contiguous()
-    fused = (mlp.lin_direct.bias is None and not any(t is None or has_tangent(t) for t in (x, *params))
-             and ops.mlp_leaky_takes(x, params[0:6:2] + params[6:], params[1:6:2]))
+    lead, rows = x.shape[:-1], x.reshape(-1, x.shape[-1]).contiguous()
+    fused = (mlp.lin_direct.bias is None and not any(t is None or has_tangent(t) for t in (rows, *params))
+             and ops.mlp_leaky_takes(rows, params[0:6:2] + params[6:], params[1:6:2]))
     if fused:
-        return _MlpLeaky.apply(x, *params).reshape(*lead, -1)
-    if mlp.lin_direct.bias is None:
-        return _mlp_leaky_rows(params, x).reshape(*lead, -1)
-    return (_mlp_leaky_rows(params, x) + mlp.lin_direct.bias).reshape(*lead, -1)
+        inside = residual and params[4].shape[0] == rows.shape[1]
+        y = _MlpLeaky.apply(inside, rows, *params).reshape(*lead, -1)
+        return x + y if residual and not inside else y
+    y = _mlp_leaky_rows(params, rows)
+    if mlp.lin_direct.bias is not None:
+        y = y + mlp.lin_direct.bias
+    y = y.reshape(*lead, -1)
+    return x + y if residual else y
 
 
 def radial_encode_painn(r, n, rmax):
@@ -1310,7 +1316,7 @@ def bee_messages(msg, graph, r_ij, x_a, x_v, x_d):
         P0, S1, S2 = _MessageProducts.apply(*nodes, enc, rh, graph.by_dst, graph.by_src,
                                             (enc8.detach(), msg.lin_enc.weight, msg.lin_enc.bias), False)
         psi_a, *sums = (_linears_of_rank(msg, k, P) for k, P in enumerate((P0, S1, S2)))
-        psi_a = psi_a + mlp_leaky(msg.mlp_a, psi_a)
+        psi_a = mlp_leaky(msg.mlp_a, psi_a, residual=True)
         return (mul(gl.edges_reduce_src(graph, psi_a), 0.1), *(mul(t.reshape(B, N, *t.shape[1:]), 0.1) for t in sums))
     prods = message_products(graph, msg.L0(x_a), msg.L1(x_v), msg.L2(x_d), enc, rh,
                              enc_source=(enc8.detach(), msg.lin_enc.weight, msg.lin_enc.bias))
@@ -1323,7 +1329,7 @@ def bee_messages(msg, graph, r_ij, x_a, x_v, x_d):
             psi_a = y if psi_a is None else psi_a + y
         else:
             sums[k] = y if sums[k] is None else sums[k] + y
-    psi_a = psi_a + mlp_leaky(msg.mlp_a, psi_a)
+    psi_a = mlp_leaky(msg.mlp_a, psi_a, residual=True)
     return mul(gl.edges_reduce_src(graph, psi_a), 0.1), mul(sums[1], 0.1), mul(sums[2], 0.1)
 
 

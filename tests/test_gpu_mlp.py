@@ -254,6 +254,29 @@ def test_biases_at_any_offset_summed_over_segments(bee, ops, monkeypatch):
         called.clear()
 
 
+@pytest.mark.parametrize("rows, dim_in, dim", [(256, 64, 64), (300, 96, 160), (5000, 256, 256)])
+def test_leaky_mlp_that_adds_its_input(ops, rows, dim_in, dim):
+    """x + mlp(x) and its gradients against the same kernels with the addition outside: one rounding more or less; a row that the pieces
+    cannot carry; sizes that differ are refused."""
+    g = torch.Generator().manual_seed(rows)
+    W = [(torch.randn(o, k, generator=g) * k ** -0.5).cuda() for o, k in ((dim, dim_in), (dim, dim), (dim_in, dim), (dim_in, dim_in))]
+    b = [(torch.randn(w.shape[0], generator=g) * 0.1).cuda() for w in W[:3]]
+    x, dy = (torch.randn(rows, dim_in, generator=g).cuda() for _ in range(2))
+    x[5] *= 2.0 ** -100
+    dy[7] *= 2.0 ** -100
+    y, saved = ops.mlp_leaky_fwd(x, W, b)
+    both, saved_both = ops.mlp_leaky_fwd(x, W, b, True)
+    _assert_rows(both, x.double() + y.double(), "x + y")
+    assert all(torch.equal(s, t) for s, t in zip(saved, saved_both))
+    g_x, params = ops.mlp_leaky_bwd(dy, x, W, saved, True, True)
+    g_both, params_both = ops.mlp_leaky_bwd(dy, x, W, saved, True, True, True)
+    _assert_rows(g_both, dy.double() + g_x.double(), "g_x")
+    assert all(torch.equal(s, t) for s, t in zip(params, params_both))
+    narrow = [W[0], W[1], W[2][:32].contiguous(), W[3][:32].contiguous()]
+    with pytest.raises(RuntimeError):
+        ops.mlp_leaky_fwd(x, narrow, [b[0], b[1], b[2][:32].contiguous()], True)
+
+
 @pytest.mark.parametrize("rows, dim_in, dim, dim_out", [(256, 64, 64, 32), (257, 96, 96, 160), (700, 256, 512, 256),
                                                          (5000, 64, 128, 64)])
 def test_leaky_mlp_and_its_adjoint(ops, rows, dim_in, dim, dim_out):
