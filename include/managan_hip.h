@@ -378,6 +378,9 @@ typedef struct mg_f16x2_linear {
 int mg_tensor_linear_f16x2_run(const mg_f16x2_linear* args /* host */, mg_stream_t stream);
 /* the same with the rows of x x_stride floats apart (a multiple of 4) */
 int mg_tensor_linear_f16x2_run_strided(const mg_f16x2_linear* args /* host */, long x_stride, mg_stream_t stream);
+/* the same for rows without bounds: their maxima are found here and written to x_rowmax_out (rows); args->x_rowmax and what belongs to it
+ * are not read */
+int mg_tensor_linear_f16x2_run_unbounded(const mg_f16x2_linear* args /* host */, float* x_rowmax_out, mg_stream_t stream);
 int mg_tensor_linear_f16x2_rowmax_parts_sequential(long rows, int dim_in, int dim_out);
 /* Linear, SiLU, Linear, SiLU, Linear (archs/meanflow_painn8.py:38-51) on plain rows as one kernel, the hidden rows staying on
  * chip: x (rows, dim_in) -> y (rows, dim), hidden layers of `dim` columns, packed_W from mg_linear_f16x2_pack_weight, biases

@@ -87,6 +87,7 @@ _SIGNATURES = {
     "mg_linear_f16x2_pack_weight": [vp, i64, i64, i32, i32, vp, vp],
     "mg_row_absmax": [vp, i64, i32, vp, vp],
     "mg_linear_f64": [vp, vp, vp, i64, i32, i32, i32, vp, vp],
+    "mg_tensor_linear_f16x2_run_unbounded": [vp, vp, vp],
     "mg_tensor_linear_f16x2_run": [vp, vp],
     "mg_tensor_linear_f16x2_run_strided": [vp, i64, vp],
     "mg_tensor_linear_f16x2_rowmax_parts_sequential": [i64, i32, i32],

@@ -223,21 +223,26 @@ int64_t rowmax_parts(int64_t rows, int64_t dim_in, int64_t dim_out, bool sequent
                       : mg_tensor_linear_f16x2_rowmax_parts(rows, (int)dim_in, (int)dim_out);
 }
 
-// x (rows, k) plain rows; y preallocated; packed: W's planes where the caller holds them
-void run_f16x2(const at::Tensor& W, int64_t k, const float* x, int64_t rows, const Bound& b, const OptTensor& bias, int act,
+// x (rows, k) plain rows; y preallocated; packed: W's planes where the caller holds them; without a base in b the rows' maxima are found on the
+// way, and returned
+OptTensor run_f16x2(const at::Tensor& W, int64_t k, const float* x, int64_t rows, const Bound& b, const OptTensor& bias, int act,
                bool accumulate, int out_comps, at::Tensor& y, at::Tensor* ymax, bool sequential, int64_t bias_rows = -1,
                const OptTensor& packed = OptTensor(), int64_t x_stride = -1, int64_t max_column = 0) {
     const at::Tensor planes = packed.has_value() ? *packed : packed_f16x2(W, k);
-    const at::Tensor& base = *b.base;
+    const bool bounded = b.base.has_value();
+    TORCH_CHECK(bounded || (x_stride < 0 && b.mul == 1.f && b.add == 0.f && b.rows_per == 1), "row maxima are found of contiguous rows");
+    at::Tensor base = bounded ? *b.base : floats(y, {rows, 1});
     mg_f16x2_linear a{};
     a.packed_W = planes.data_ptr();
     a.x = x;
-    a.x_rowmax = fp(base) + max_column;                        // (x_stride: a column of `base` for each block of columns of x)
-    a.x_rowmax_parts = x_stride < 0 ? (int)base.size(1) : 1;
-    a.x_rowmax_stride = base.size(0) > 1 || rows == b.rows_per ? base.size(1) : 0;
-    a.x_rows_per_bound = b.rows_per;
-    a.bound_mul = b.mul;
-    a.bound_add = b.add;
+    if (bounded) {
+        a.x_rowmax = fp(base) + max_column;                    // (x_stride: a column of `base` for each block of columns of x)
+        a.x_rowmax_parts = x_stride < 0 ? (int)base.size(1) : 1;
+        a.x_rowmax_stride = base.size(0) > 1 || rows == b.rows_per ? base.size(1) : 0;
+        a.x_rows_per_bound = b.rows_per;
+        a.bound_mul = b.mul;
+        a.bound_add = b.add;
+    }
     a.rows = rows;
     a.dim_in = (int)k;
     a.dim_out = (int)W.size(0);
@@ -249,7 +254,9 @@ void run_f16x2(const at::Tensor& W, int64_t k, const float* x, int64_t rows, con
     a.sequential = sequential;
     a.y = fp(y);
     a.y_rowmax = ymax ? fp(*ymax) : nullptr;
-    check(mg_tensor_linear_f16x2_run_strided(&a, x_stride < 0 ? k : x_stride, stream_of(y)));
+    if (bounded) check(mg_tensor_linear_f16x2_run_strided(&a, x_stride < 0 ? k : x_stride, stream_of(y)));
+    else check(mg_tensor_linear_f16x2_run_unbounded(&a, fp(base), stream_of(y)));
+    return base;
 }
 
 void check_bound(const at::Tensor& b, int64_t rows, int64_t rows_per) {
@@ -395,12 +402,11 @@ std::tuple<at::Tensor, OptTensor> linear_fwd(int64_t inds, const at::Tensor& W, 
         }
         run_f16x2(W, k_pad, fp(x2), R, Bound{x2max}, bias, act, accumulate, out_comps, y, rowmax_buffer(k_pad), sequential);
     } else if (plain_rows && mode == kModeF16x2 && f16x2_takes(R, dim_in, dim_out, x) && (!sequential || R >= 256)) {
-        Bound b{row_bound, (float)mul, (float)add, rows_per};
+        Bound b;
         if (row_bound.has_value()) {
+            b = Bound{row_bound, (float)mul, (float)add, rows_per};
             TORCH_CHECK(row_bound->dim() == 2 && (row_bound->size(0) * rows_per == R || row_bound->size(0) == 1),
                         "row_bound must be (rows / rows_per_bound, parts)");
-        } else {
-            b = Bound{row_absmax(x.reshape({R, dim_in}))};
         }
         run_f16x2(W, dim_in, fp(x), R, b, bias, act, accumulate, out_comps, y, rowmax_buffer(dim_in), sequential);
     } else if (mode == kModeBf16x3 && plain_rows && dim_in % 32 == 0 && dim_in >= 64 && dim_out >= 64 && R >= 1024 &&
@@ -575,8 +581,8 @@ at::Tensor chain(at::Tensor h, const Tensors& W, const Tensors& b, const std::ve
             continue;
         }
         if (mg_get_linear_mode() == kModeF16x2 && f16x2_takes(rows, dim_in, dim_out, h)) {
-            if (!bound.base.has_value()) bound = Bound{row_absmax(h)};
-            run_f16x2(W[k], dim_in, fp(h), rows, bound, bias, act[k], false, 1, y, nullptr, false);
+            if (!bound.base.has_value()) bound = Bound{};
+            bound.base = run_f16x2(W[k], dim_in, fp(h), rows, bound, bias, act[k], false, 1, y, nullptr, false);
         } else {
             y = std::get<0>(linear_fwd(0, W[k], h, bias, act[k], OptTensor(y), false, 0, 0, OptTensor(), 1, 0, 1, false,
                                        OptTensor(), OptTensor(), false));
@@ -995,7 +1001,7 @@ at::Tensor rows_linear(const at::Tensor& W, const OptTensor& bias, const at::Ten
     at::Tensor y = floats(x, {rows, dim_out});
     if (rows == 0) return y;
     if (mg_get_linear_mode() == kModeF16x2 && f16x2_takes(rows, dim_in, dim_out, x)) {
-        if (!bound.base.has_value()) bound = Bound{row_absmax(x)};
+        if (!bound.base.has_value()) bound = Bound{};
         run_f16x2(W, dim_in, fp(x), rows, bound, bias, kActNone, false, 1, y, nullptr, false, bias_rows, packed);
         return y;
     }

@@ -622,6 +622,26 @@ def test_weight_gradient_with_one_narrow_dimension(ops, inds, rows, dims):
     assert not marked[0].isfinite().any() and torch.equal(marked[1:], dW[1:])
 
 
+@pytest.mark.parametrize("rows,dim_in,dim_out", [(1, 64, 64), (33, 128, 512), (337, 512, 512), (300, 1280, 96), (2048, 256, 256),
+                                                 (40, 96, 40), (60000, 64, 128)])
+def test_linear_that_finds_its_own_row_maxima(ops, rows, dim_in, dim_out):
+    """Without bounds the results are those with the exact row maxima to the bit, on either side of the line to reductions split over
+    waves, fewer pieces of a row than waves and more; a layer behind it scales by the maxima that it wrote.  Rows of zeros, of small
+    numbers, with infinities and NaN."""
+    g = torch.Generator().manual_seed(rows + dim_in)
+    W, b = (torch.randn(dim_out, dim_in, generator=g) * dim_in ** -0.5).cuda(), torch.randn(dim_out, generator=g).cuda()
+    W2, b2 = (torch.randn(dim_out, dim_out, generator=g) * dim_out ** -0.5).cuda(), torch.randn(dim_out, generator=g).cuda()
+    x = torch.randn(rows, dim_in, generator=g) * torch.randint(-20, 20, (rows, 1), generator=g).float().exp2()
+    if rows > 30:
+        x[3], x[5, 7], x[9, dim_in - 1], x[11] = 0.0, float("inf"), float("nan"), x[11] * 2.0 ** -120
+    x = x.cuda()
+    bound = ops.row_absmax(x)
+    same = lambda a, b: torch.equal(a.nan_to_num(1.5), b.nan_to_num(1.5))
+    assert same(ops.tensor_linear_fwd(0, W, x, bias=b), ops.tensor_linear_fwd(0, W, x, bias=b, row_bound=bound))
+    acts = [ops.ACT_SILU, ops.ACT_NONE]
+    assert same(ops._ext.linear_chain(x, [W, W2], [b, b2], acts, None, 1.0, 0.0), ops._ext.linear_chain(x, [W, W2], [b, b2], acts, bound, 1.0, 0.0))
+
+
 class _WgradJob(ctypes.Structure):
     _fields_ = [("dy", ctypes.c_void_p), ("x", ctypes.c_void_p), ("dy_bound", ctypes.c_void_p), ("n_dy_bound", ctypes.c_long),
                 ("x_bound", ctypes.c_void_p), ("n_x_bound", ctypes.c_long), ("bias_rows", ctypes.c_long), ("dim_in", ctypes.c_int),
