@@ -948,6 +948,11 @@ int mg_painn_update_pre(const float* lrv, int lrv_comp_major, const float* x_a, 
 /* (lrv_comp_major = 2: lrv is lin_v(x_v) alone, (rows, 3, n)) */
 int mg_painn_update_vec(const float* lrv, int lrv_comp_major, const float* y, const float* res_v /* or NULL */, long rows, int n,
                         float* out_v, mg_stream_t stream);
+/* The group norm and the vector output of an Update in one pass: out_a = groupnorm(ip y[n:2n]) + y[2n:3n] [+ res_a], out_v as
+ * mg_painn_update_vec; rows = batch x nodes, scratch as mg_group_norm. */
+int mg_painn_update_post(const float* lrv, int lrv_comp_major, const float* ip, const float* y, int batch, int nodes, int n, int groups,
+                         float eps, const float* gamma, const float* beta, const float* res_a, const float* res_v, void* scratch,
+                         float* out_a, float* out_v, mg_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Norms, squash, remaining radial encodings (node- or edge-sized streaming kernels).

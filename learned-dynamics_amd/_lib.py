@@ -115,6 +115,7 @@ _SIGNATURES = {
     "mg_painn_update_maps_supported": [i32],
     "mg_painn_update_maps": [vp, vp, i64, i32, vp, vp, vp, vp, vp, vp],
     "mg_painn_update_pre": [vp, i32, vp, i64, i32, vp, vp, vp, vp],
+    "mg_painn_update_post": [vp, i32, vp, vp, i32, i32, i32, i32, f32, vp, vp, vp, vp, vp, vp, vp, vp],
     "mg_painn_update_vec": [vp, i32, vp, vp, i64, i32, vp, vp],
     "mg_radial_encode": [i32, vp, i64, i32, f32, vp, vp],
     "mg_bee_node_products": [i64, i32, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp],

@@ -94,6 +94,29 @@ __device__ __forceinline__ float2 fold_group(const double* __restrict__ partial,
     return make_float2((float)mean, sqrtf(eps + (float)var));
 }
 
+template <bool COMP_MAJOR>
+__device__ __forceinline__ float lrv_at(const float* __restrict__ row, int n, int j, int x) {
+    return COMP_MAJOR ? row[x * 3 * n + j] : row[j * 3 + x];
+}
+
+// PaiNN Update, vector output: v = lin_v(x_v) * y[0:n]; out = res_v + v / sqrt(1 + |v|^2), out (rows, n, 3).  LAYOUT: of lrv, as
+// lrv_comp_major of mg_painn_update_vec
+struct UpdateVec {
+    const float *lrv, *y, *res_v;
+    float* out_v;
+};
+template <int LAYOUT>
+__device__ __forceinline__ void update_vec(const UpdateVec& a, long r, int n, int c) {
+    const float s = a.y[r * 3 * n + c];
+    auto v_at = [&](int x) { return LAYOUT == 2 ? a.lrv[(r * 3 + x) * n + c] : lrv_at<LAYOUT == 1>(a.lrv + r * 9 * n, n, 2 * n + c, x); };
+    const float v0 = v_at(0) * s, v1 = v_at(1) * s, v2 = v_at(2) * s;
+    const float inv = 1.0f / sqrtf(1.0f + (v0 * v0 + v1 * v1 + v2 * v2));
+    float o0 = v0 * inv, o1 = v1 * inv, o2 = v2 * inv;
+    const long t = 3 * (r * n + c);
+    if (a.res_v) { o0 += a.res_v[t]; o1 += a.res_v[t + 1]; o2 += a.res_v[t + 2]; }
+    a.out_v[t] = o0; a.out_v[t + 1] = o1; a.out_v[t + 2] = o2;
+}
+
 // mode 0 (TensGroupNorm): y = gamma[c] * v / sqrt(eps + mean(sum_comp v^2))
 // mode 1 (ScalGroupNorm, T = 1): y = beta[c] + gamma[c] * (v - mean) / sqrt(eps + var)
 // then y += add (optional, add_stride) and y += res (optional, same layout as out).
@@ -101,13 +124,17 @@ __device__ __forceinline__ float2 fold_group(const double* __restrict__ partial,
 // nodes: channel, group, gamma, beta and the group's statistics are fixed per thread, consecutive threads touch
 // consecutive floats.  A workgroup folds the partial sums of the groups that its positions belong to by itself (a launch for it took
 // 3 us on one system and 5 on 32 of them; each node array had one).
+// VEC: the vector output of a PaiNN Update, whose rows have as many channels, beside it (layout VEC - 1): 16 336 nodes of
+// 128 channels 22.5 us, 26.0 in two launches, 337 nodes 9.7, 9.6 and a launch.
+template <int VEC = 0>
 __global__ void __launch_bounds__(256) group_apply_kernel(const float* __restrict__ x, long x_stride,
                                                           const float* __restrict__ mul, long mul_stride,
                                                           const double* __restrict__ partial, int N, int chan,
                                                           int groups, int T, int mode, float eps,
                                                           const float* __restrict__ gamma, const float* __restrict__ beta,
                                                           const float* __restrict__ add, long add_stride,
-                                                          const float* __restrict__ res, float* __restrict__ out) {
+                                                          const float* __restrict__ res, float* __restrict__ out,
+                                                          const UpdateVec vec) {
     __shared__ float2 stats[256];                                  // (a position a thread: no more groups than that)
     const int CT = chan * T, b = blockIdx.z, per = chan / groups * T;
     const int k_first = blockIdx.x * blockDim.x, k = k_first + (int)threadIdx.x;
@@ -144,6 +171,8 @@ __global__ void __launch_bounds__(256) group_apply_kernel(const float* __restric
             const int node = i + u * (int)gridDim.y;
             const float y = mode == 0 ? ga * (v[u] / denom) : be + ga * ((v[u] - mean) / denom);
             if (node < N) out[((long)b * N + node) * CT + k] = y + plus[u];
+            if constexpr (VEC != 0)
+                if (node < N) update_vec<VEC - 1>(vec, (long)b * N + node, CT, k);
         }
     }
 }
@@ -233,11 +262,6 @@ __global__ void __launch_bounds__(256) tens_sigmoid_kernel(const float* __restri
 // (rows, 3, 3n) (what the GEMM stores at full rate, and what a wave reads here with unit stride)
 //   ip[r,c] = sum_x l[c,x] r[c,x];  cat[r] = [x_a[r] | |r[c]|]   (rows, 2n)
 // One workgroup row per node row: blockIdx.x = r, the channel from blockIdx.y and the thread.
-template <bool COMP_MAJOR>
-__device__ __forceinline__ float lrv_at(const float* __restrict__ row, int n, int j, int x) {
-    return COMP_MAJOR ? row[x * 3 * n + j] : row[j * 3 + x];
-}
-
 // cat_rowmax (rows; or null): max |cat[r, :]|, the row bound of the MLP that reads cat; written when one workgroup
 // covers a row (n <= 256: gridDim.y == 1)
 template <bool COMP_MAJOR>
@@ -270,23 +294,10 @@ __global__ void __launch_bounds__(256) painn_update_pre_kernel(const float* __re
     }
 }
 
-// PaiNN Update, vector output: v = lin_v(x_v) * y[0:n]; out = res_v + v / sqrt(1 + |v|^2), out (rows, n, 3).  LAYOUT: of lrv, as
-// lrv_comp_major of mg_painn_update_vec
 template <int LAYOUT>
-__global__ void __launch_bounds__(256) painn_update_vec_kernel(const float* __restrict__ lrv, const float* __restrict__ y,
-                                                               const float* __restrict__ res_v, int n,
-                                                               float* __restrict__ out_v) {
-    const long r = blockIdx.x;
+__global__ void __launch_bounds__(256) painn_update_vec_kernel(const UpdateVec a, int n) {
     const int c = blockIdx.y * blockDim.x + threadIdx.x;
-    if (c >= n) return;
-    const float s = y[r * 3 * n + c];
-    auto v_at = [&](int x) { return LAYOUT == 2 ? lrv[(r * 3 + x) * n + c] : lrv_at<LAYOUT == 1>(lrv + r * 9 * n, n, 2 * n + c, x); };
-    const float a = v_at(0) * s, b = v_at(1) * s, d = v_at(2) * s;
-    const float inv = 1.0f / sqrtf(1.0f + (a * a + b * b + d * d));
-    float o0 = a * inv, o1 = b * inv, o2 = d * inv;
-    const long t = r * n + c;
-    if (res_v) { o0 += res_v[3 * t]; o1 += res_v[3 * t + 1]; o2 += res_v[3 * t + 2]; }
-    out_v[3 * t] = o0; out_v[3 * t + 1] = o1; out_v[3 * t + 2] = o2;
+    if (c < n) update_vec<LAYOUT>(a, blockIdx.x, n, c);
 }
 
 // kinds: 1 sq_radial_encode of normed_sq_dist (archs/diffuser_atoms14.py:32-48)
@@ -341,9 +352,10 @@ static dim3 apply_grid(int batch, int nodes, int CT, int* threads) {
     return dim3((unsigned)kx, (unsigned)ny, (unsigned)batch);
 }
 
-int mg_group_norm(int mode, const float* x, long x_stride, const float* mul, long mul_stride, int batch, int nodes,
-                  int chan, int groups, int comps, float eps, const float* gamma, const float* beta, const float* add,
-                  long add_stride, const float* res, void* scratch, float* out, mg_stream_t stream) {
+// vec: 0, or 1 + the layout of `with`, the vector output written beside it
+static int group_norm(int mode, const float* x, long x_stride, const float* mul, long mul_stride, int batch, int nodes, int chan, int groups,
+                      int comps, float eps, const float* gamma, const float* beta, const float* add, long add_stride, const float* res,
+                      void* scratch, float* out, int vec, const UpdateVec& with, mg_stream_t stream) {
     MG_REQUIRE(mode == 0 || mode == 1, "mg_group_norm: mode must be 0 (tensor) or 1 (scalar)");
     MG_REQUIRE(batch >= 0 && nodes >= 0 && chan >= 0 && groups > 0 && chan % groups == 0, "mg_group_norm: bad sizes");
     MG_REQUIRE(comps == 1 || comps == 3 || comps == 9, "mg_group_norm: comps must be 1, 3 or 9");
@@ -357,10 +369,26 @@ int mg_group_norm(int mode, const float* x, long x_stride, const float* mul, lon
                        mul_stride, nodes, chan, groups, comps, static_cast<double*>(scratch));
     int threads;
     const dim3 grid = apply_grid(batch, nodes, chan * comps, &threads);
-    hipLaunchKernelGGL(group_apply_kernel, grid, dim3(threads), 0, st, x,
-                       x_stride, mul, mul_stride, static_cast<const double*>(scratch), nodes, chan, groups, comps, mode, eps,
-                       gamma, beta, add, add_stride, res, out);
+    const auto kernel = vec == 0 ? group_apply_kernel<0> : vec == 1 ? group_apply_kernel<1> : vec == 2 ? group_apply_kernel<2> : group_apply_kernel<3>;
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, st, x, x_stride, mul, mul_stride, static_cast<const double*>(scratch), nodes, chan,
+                       groups, comps, mode, eps, gamma, beta, add, add_stride, res, out, with);
     return check_launch("mg_group_norm");
+}
+
+int mg_group_norm(int mode, const float* x, long x_stride, const float* mul, long mul_stride, int batch, int nodes,
+                  int chan, int groups, int comps, float eps, const float* gamma, const float* beta, const float* add,
+                  long add_stride, const float* res, void* scratch, float* out, mg_stream_t stream) {
+    return group_norm(mode, x, x_stride, mul, mul_stride, batch, nodes, chan, groups, comps, eps, gamma, beta, add, add_stride, res, scratch,
+                      out, 0, UpdateVec{}, stream);
+}
+
+int mg_painn_update_post(const float* lrv, int lrv_comp_major, const float* ip, const float* y, int batch, int nodes, int n, int groups,
+                         float eps, const float* gamma, const float* beta, const float* res_a, const float* res_v, void* scratch,
+                         float* out_a, float* out_v, mg_stream_t stream) {
+    MG_REQUIRE(lrv_comp_major >= 0 && lrv_comp_major <= 2, "mg_painn_update_post: lrv_comp_major must be 0, 1 or 2");
+    MG_REQUIRE((long)batch * nodes * n == 0 || (lrv && y && ip && out_v), "mg_painn_update_post: null pointer");
+    return group_norm(1, ip, n, y + n, 3L * n, batch, nodes, n, groups, 1, eps, gamma, beta, y + 2 * n, 3L * n, res_a, scratch, out_a,
+                      1 + lrv_comp_major, UpdateVec{lrv, y, res_v, out_v}, stream);
 }
 
 int mg_tensor_norm_grad_workspace_bytes(int batch, int chan, int groups, int comps, size_t* bytes) {
@@ -427,7 +455,7 @@ int mg_painn_update_vec(const float* lrv, int lrv_comp_major, const float* y, co
     const int threads = n >= 256 ? 256 : (int)ceil_div(n, kWave) * kWave;
     const dim3 grid((unsigned)rows, (unsigned)ceil_div(n, threads));
     const auto kernel = lrv_comp_major == 2 ? painn_update_vec_kernel<2> : (lrv_comp_major ? painn_update_vec_kernel<1> : painn_update_vec_kernel<0>);
-    hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, (hipStream_t)stream, lrv, y, res_v, n, out_v);
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, (hipStream_t)stream, UpdateVec{lrv, y, res_v, out_v}, n);
     return check_launch("mg_painn_update_vec");
 }
 

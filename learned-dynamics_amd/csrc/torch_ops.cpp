@@ -651,9 +651,8 @@ std::tuple<at::Tensor, at::Tensor> painn_update(const at::Tensor& x_a, const at:
     size_t scratch_bytes = 0;
     check(mg_group_norm_scratch_bytes((int)B, groups, &scratch_bytes));
     at::Tensor scratch = bytes_like(x_a, std::max<size_t>(scratch_bytes, 8));
-    check(mg_group_norm(1, fp(ip), n, fp(y) + n, 3 * n, (int)B, (int)N, (int)n, groups, 1, (float)eps, fp(gamma), fp(beta),
-                        fp(y) + 2 * n, 3 * n, residual ? fp(x_a) : nullptr, scratch.data_ptr(), fp(out_a), st));
-    check(mg_painn_update_vec(fp(lrv), maps ? 2 : 1, fp(y), residual ? fp(x_v) : nullptr, rows, (int)n, fp(out_v), st));
+    check(mg_painn_update_post(fp(lrv), maps ? 2 : 1, fp(ip), fp(y), (int)B, (int)N, (int)n, groups, (float)eps, fp(gamma), fp(beta),
+                               residual ? fp(x_a) : nullptr, residual ? fp(x_v) : nullptr, scratch.data_ptr(), fp(out_a), fp(out_v), st));
     return {out_a, out_v};
 }
 

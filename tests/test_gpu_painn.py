@@ -3,6 +3,7 @@ against the oracle's restatement of archs/meanflow_painn8.py.
 
 Tolerance (tests/parity.py): rel 1e-5 / abs 1e-6 against the formula in float64, widened only by twice the distance of
 the same formula evaluated in float32 from it."""
+import ctypes
 import importlib
 
 import numpy as np
@@ -771,3 +772,28 @@ def test_update_with_its_maps_in_one_kernel(pkg, rows, n):
     assert torch.equal(odd[0, keep], got[1][0, keep])
     # (|r|^2 of both rows is beyond 2^128: undefined as from any sum of squares in fp32)
     assert not bool(torch.isfinite(odd[0, ~keep]).any())
+
+
+@pytest.mark.parametrize("batch,nodes,n,groups", [(1, 1, 4, 1), (2, 337, 128, 4), (1, 5, 300, 3), (3, 1000, 64, 4)])
+@pytest.mark.parametrize("layout", [0, 1, 2])
+def test_group_norm_and_vector_output_in_one_pass(ops, batch, nodes, n, groups, layout):
+    """mg_painn_update_post against mg_group_norm and mg_painn_update_vec: the same bits, with rows to add and without, channels of more
+    than one workgroup, every layout of the maps."""
+    L = importlib.import_module("learned-dynamics_amd._lib")
+    lib, g = L.load(), torch.Generator(device="cuda").manual_seed(nodes + n)
+    rows, stream = batch * nodes, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    lrv, ip, y, gamma, beta, x_a, x_v = rnd(rows, 9 * n), rnd(rows, n), rnd(rows, 3 * n), rnd(n), rnd(n), rnd(rows, n), rnd(rows, 3 * n)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    size = ctypes.c_size_t()
+    L.check(lib.mg_group_norm_scratch_bytes(batch, groups, ctypes.byref(size)))
+    scratch = torch.empty(size.value, dtype=torch.uint8, device="cuda")
+    for res_a, res_v in ((None, None), (p(x_a), p(x_v))):
+        out = [rnd(rows, n), rnd(rows, 3 * n), rnd(rows, n), rnd(rows, 3 * n)]
+        y2, y3 = (ctypes.c_void_p(y.data_ptr() + 4 * k * n) for k in (1, 2))
+        L.check(lib.mg_group_norm(1, p(ip), n, y2, 3 * n, batch, nodes, n, groups, 1, 1.0, p(gamma), p(beta), y3, 3 * n, res_a, p(scratch),
+                                  p(out[0]), stream))
+        L.check(lib.mg_painn_update_vec(p(lrv), layout, p(y), res_v, rows, n, p(out[1]), stream))
+        L.check(lib.mg_painn_update_post(p(lrv), layout, p(ip), p(y), batch, nodes, n, groups, 1.0, p(gamma), p(beta), res_a, res_v,
+                                         p(scratch), p(out[2]), p(out[3]), stream))
+        assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[3])
