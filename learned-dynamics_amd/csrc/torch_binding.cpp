@@ -373,7 +373,12 @@ torch::autograd::variable_list TensorLinearFn::backward(torch::autograd::Autogra
     return {at::Tensor(), dW, dx};
 }
 
-at::Tensor tensor_linear(int64_t inds, const at::Tensor& W, const at::Tensor& x) { return TensorLinearFn::apply(inds, W, x); }
+at::Tensor tensor_linear(int64_t inds, const at::Tensor& W, const at::Tensor& x) {
+    // with nothing to record and no tangent to refuse, the function's bookkeeping would be a third of the call's host time
+    const bool recorded = at::GradMode::is_enabled() && (W.requires_grad() || x.requires_grad());
+    if (!recorded && !W._fw_grad(0).defined() && !x._fw_grad(0).defined()) return linear_forward(inds, W, x);
+    return TensorLinearFn::apply(inds, W, x);
+}
 
 // ------------------------------------------------------------------ TensorProds in one launch
 // y = lin_o(prod(lin_l(x_l), lin_r(x_r))) (managan/tensor_products.py:109-121), for problems mg_tensor_prods_supported
