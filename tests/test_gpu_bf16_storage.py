@@ -311,3 +311,10 @@ def test_tens_group_norm_bf16(ops, comps, chan, groups, with_res):
     assert float((err > 1.001 * half_ulp + fp32_noise).double().mean()) < 0.01       # almost always correctly rounded
     with pytest.raises(RuntimeError, match="multiple of 8"):
         ops.tens_group_norm_bf16(torch.zeros(4, 12, dtype=torch.bfloat16, device="cuda"), 1, 4, torch.ones(12, device="cuda"), eps)
+
+
+@pytest.mark.parametrize("comps,chan,groups", [(1, 8, 8), (1, 24, 24), (3, 40, 5), (9, 8, 1), (1, 2048, 256), (1, 2056, 8)])
+def test_tens_group_norm_bf16_where_columns_and_threads_do_not_divide(ops, comps, chan, groups):
+    """Rows that leave threads of the statistics pass without a column (a row of one 16-byte piece, of 15), groups that 256
+    threads do not divide by, one thread to a group, and one piece more than a workgroup has threads."""
+    test_tens_group_norm_bf16(ops, comps, chan, groups, False)
