@@ -626,26 +626,29 @@ __global__ void __launch_bounds__(256) wgrad_reduce_kernel(const float* __restri
     }
 }
 
-// Sums of planes of few quads and many slices: 16 threads a quad, whose sums are added in their order: one
-// thread a quad took 10 to 13 us for planes of 1000 quads and 192 to 512 slices, four workgroups, of which each load is waited for.
+// Sums of planes of few quads and many slices: 16 threads a quad, every sum in pairs (512 slices one after the other were a third
+// of a narrow gradient's rounding): one thread a quad took 10 to 13 us for planes of 1000 quads and 192 to 512 slices, four workgroups, of which each load is waited for.
 __device__ __forceinline__ float4 sum_of_slices(const float4* __restrict__ part, int quads, int splits, int k, float4* shared) {
     const int z = threadIdx.x >> 4;
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto plus = [](const float4& a, const float4& b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); };
     auto add = [&](const float4& v) { s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w; };
     if (k < quads) {
         int j = z;
         for (; j + 48 < splits; j += 64) {
             const float4 v0 = part[(long)j * quads + k], v1 = part[(long)(j + 16) * quads + k], v2 = part[(long)(j + 32) * quads + k],
                          v3 = part[(long)(j + 48) * quads + k];
-            add(v0); add(v1); add(v2); add(v3);
+            add(plus(plus(v0, v1), plus(v2, v3)));
         }
         for (; j < splits; j += 16) add(part[(long)j * quads + k]);
     }
     shared[threadIdx.x] = s;
     __syncthreads();
-    s = shared[threadIdx.x & 15];
-    for (int j = 1; j < 16; j++) add(shared[16 * j + (threadIdx.x & 15)]);
-    return s;
+    const float4* of = shared + (threadIdx.x & 15);
+    float4 four[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) four[j] = plus(plus(of[64 * j], of[64 * j + 16]), plus(of[64 * j + 32], of[64 * j + 48]));
+    return plus(plus(four[0], four[1]), plus(four[2], four[3]));
 }
 // the same for the planes of several products: quad k of a plane goes to the segment that holds it
 struct WgradSegments {
@@ -685,21 +688,137 @@ __global__ void __launch_bounds__(256) wgrad_reduce_f16x2_kernel(const float4* _
 }
 
 // ---------------------------------------------------------------------------------------- one dimension of at most 16
-// P[k, i] = sum_{r, t} narrow[r, k, t] wide[r, i, t] with k < n <= 16: two to thirty-two multiply-adds a float of the wide operand, which
+// P[k, i] = sum_{r, t} narrow[r, k, t] wide[r, i, t] with k < n <= 16: two to thirty-two operations a float of the wide operand, which
 // is read once, 16 bytes a lane, in whatever layout of components it has: nothing is transposed, and products and sums are fp32, so
-// no bounds are needed either.  A lane holds the n results of four channels, L lanes a row, 256 / L rows at a time; the narrow
-// operand's rows lie in LDS, where all lanes of a row read the same words.
-// Bound by memory: 1.5 M rows 16 -> 512 at 4.5 TB/s.  Against the split-fp16 product with its padding to 128 x 128, its row maxima and,
-// for tensors, its transposed copies: that one 1242 -> 697 us, 73 728 rows 1280 -> 16 168 -> 107, 16 -> 256 52 -> 29, 8192 rows of
-// three components 1 -> 128 and 128 -> 1 42 -> 8, 128 -> 16 41 -> 18, of nine 128 -> 1 68 -> 11.
-// BIAS: the sums of the columns of dy as well (of plain rows), where dy is the wide operand or the narrow one; behind the plane (n, dim).
-constexpr int kNarrow = 16, kNarrowRows = 64;
+// no bounds are needed either.
+constexpr int kNarrow = 16, kNarrowRows = 64, kNarrowChains = 4;
 enum NarrowBias { kNoBias, kOfWide, kOfNarrow };
-template <int T, int N, int BIAS = kNoBias>
+
+// Plain rows, by matrix instructions: a wave takes 64 channels of every (4 / waves_c)-th step of four rows, a lane one row and four
+// channels of the wide operand and one number of the narrow one, both as they lie in memory.  No LDS and no barrier until the end,
+// so loads of kAhead steps are in flight while the steps before them are multiplied; the sums of every fourth step are a chain of
+// their own (64 registers, and no longer chains than sixteen groups of lanes would have).
+// Bound by memory: 1.5 M rows 16 -> 512 at 5.8 TB/s, 73 728 rows 1280 -> 16 at 5.0.  With the n results of four channels as
+// multiply-adds of one lane, the narrow rows in LDS and two barriers for every 64 rows, loads and arithmetic took turns: 697 us against
+// 545, 106 against 76, 73 728 rows 16 -> 256 32.5 against 25.5, 8192 rows 260 -> 16 15.5 against 10.3, level at 9.5 for 4096 rows
+// 64 -> 1.  The split-fp16 product with its padding to 128 x 128 and its row maxima: 1242, 168 and 52 us.  Error against float64
+// (2-norm, normal numbers): 73 728 rows 16 -> 256 1.4e-7 against 1.8e-7, 131 072 rows 8 -> 512 1.7e-7 against 2.0e-7.
+// BIAS: the sums of the columns of dy as well, where dy is the wide operand or the narrow one; behind the plane (n, dim).
+template <int BIAS>
+__global__ void __launch_bounds__(256, 4) wgrad_narrow_rows_kernel(const float* __restrict__ narrow, int n, const float* __restrict__ wide,
+                                                                int dim, long R, long rows_per_block, int waves_c, long plane,
+                                                                float* __restrict__ part) {
+    typedef float floatx4 __attribute__((ext_vector_type(4)));
+    constexpr int kAhead = BIAS == kOfWide ? 4 : 8;             // (128 registers, four workgroups on a compute unit)
+    __shared__ float4 shared[3 * 64 * 5];                      // of the row waves but the first: results, sums of columns
+    __shared__ float shared_narrow[3 * 16];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, sub = lane >> 4;
+    const int shift = __builtin_ctz(waves_c), waves_r = 4 >> shift, wr = wave >> shift, wc = wave & (waves_c - 1);
+    const int quad = (blockIdx.x * waves_c + wc) * 16 + c;
+    const bool live = quad < dim / 4;
+    const int own = live ? 4 * quad : 0, own_n = c < n ? c : 0;
+    const long r_first = (long)blockIdx.y * rows_per_block, r_hi = r_first + rows_per_block < R ? r_first + rows_per_block : R;
+    const int stride = 4 * waves_r;                            // rows between the steps of a wave
+    floatx4 acc[kNarrowChains][4];
+#pragma unroll
+    for (int u = 0; u < kNarrowChains; u++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[u][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    float column[4] = {0.f, 0.f, 0.f, 0.f};                    // BIAS: of the wide operand's four channels, or four chains of the narrow's
+    float4 x[kAhead];
+    float a[kAhead];
+    auto load = [&](int u, long r) {                           // of rows r .. r + 3; those behind the last: the last, not counted
+        const long row = r < r_hi ? r : r_hi - 1;
+        const int past = r_hi - 1 - row < 3 ? (int)(r_hi - 1 - row) : 3, k = sub < past ? sub : past;
+        x[u] = *reinterpret_cast<const float4*>(wide + row * dim + (unsigned)(k * dim + own));
+        a[u] = (narrow + row * n)[(unsigned)(k * n + own_n)];
+    };
+    auto use = [&](int u, long r) {
+        const bool in = sub < r_hi - r;                        // both operands are cleared: infinities of a row read twice stay out
+        const float v[4] = {in ? x[u].x : 0.f, in ? x[u].y : 0.f, in ? x[u].z : 0.f, in ? x[u].w : 0.f};
+        const float k = in && c < n ? a[u] : 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            acc[u % kNarrowChains][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(k, v[j], acc[u % kNarrowChains][j], 0, 0, 0);
+        if constexpr (BIAS == kOfWide)
+#pragma unroll
+            for (int j = 0; j < 4; j++) column[j] += v[j];
+        if constexpr (BIAS == kOfNarrow) column[u % 4] += k;
+    };
+    const long round = (long)kAhead * stride;
+    const int rounds = (int)((r_hi - r_first + round - 1) / round);
+    long r = r_first + 4 * wr;
+#pragma unroll
+    for (int u = 0; u < kAhead; u++) load(u, r + u * stride);
+    for (int k = 1; k < rounds; k++, r += round) {
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) {
+            use(u, r + u * stride);
+            load(u, r + round + u * stride);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; u++)
+        if (r + u * stride < r_hi) use(u, r + u * stride);      // (uniform)
+    // the chains, then the waves of rows, added in their order; a lane has the results 4 sub + i of its four channels
+    float4 sum[5];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = (acc[0][j][i] + acc[1][j][i]) + (acc[2][j][i] + acc[3][j][i]);
+        sum[i] = make_float4(v[0], v[1], v[2], v[3]);
+    }
+    constexpr int kSums = BIAS == kOfWide ? 5 : 4;
+    float of_narrow = 0.f;
+    if constexpr (BIAS == kOfWide) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            column[j] += __shfl_xor(column[j], 16);
+            column[j] += __shfl_xor(column[j], 32);
+        }
+        sum[4] = make_float4(column[0], column[1], column[2], column[3]);
+    }
+    if constexpr (BIAS == kOfNarrow) {
+        of_narrow = (column[0] + column[1]) + (column[2] + column[3]);
+        of_narrow += __shfl_xor(of_narrow, 16);
+        of_narrow += __shfl_xor(of_narrow, 32);
+    }
+    if (wr > 0) {
+        const int slot = (wr - 1) * waves_c + wc;
+#pragma unroll
+        for (int i = 0; i < kSums; i++) shared[(slot * 5 + i) * 64 + lane] = sum[i];
+        if (BIAS == kOfNarrow && wc == 0 && lane < 16) shared_narrow[(wr - 1) * 16 + c] = of_narrow;
+    }
+    __syncthreads();
+    if (wr > 0) return;
+    for (int g = 0; g < waves_r - 1; g++) {
+        const int slot = g * waves_c + wc;
+#pragma unroll
+        for (int i = 0; i < kSums; i++) {
+            const float4 v = shared[(slot * 5 + i) * 64 + lane];
+            sum[i].x += v.x; sum[i].y += v.y; sum[i].z += v.z; sum[i].w += v.w;
+        }
+        if constexpr (BIAS == kOfNarrow) of_narrow += shared_narrow[g * 16 + c];
+    }
+    float* out = part + blockIdx.y * plane;
+    if (live) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (4 * sub + i < n) *reinterpret_cast<float4*>(out + (long)(4 * sub + i) * dim + 4 * quad) = sum[i];
+        if (BIAS == kOfWide && sub == 0) *reinterpret_cast<float4*>(out + (long)n * dim + 4 * quad) = sum[4];
+    }
+    if (BIAS == kOfNarrow && blockIdx.x == 0 && wc == 0 && lane < 16) out[(long)n * dim + c] = of_narrow;
+}
+
+// Rows of T = 3 or 9 components: a lane holds the n results of four channels, L lanes a row, 256 / L rows at a time; the narrow
+// operand's rows lie in LDS, where all lanes of a row read the same words.  8192 rows of three components 1 -> 128 and 128 -> 1 8 us,
+// 128 -> 16 18, of nine 128 -> 1 11; the split-fp16 product with its padding to 128 x 128, its row maxima and transposed copies 42, 41, 68.
+template <int T, int N>
 __global__ void __launch_bounds__(256) wgrad_narrow_kernel(const float* __restrict__ narrow, int n, const float* __restrict__ wide,
                                                            int dim, long R, long rows_per_block, int L, long plane,
                                                            float* __restrict__ part) {
-    constexpr int kAhead = T == 1 ? 8 : T == 3 ? 4 : 1;       // rows requested together
+    constexpr int kAhead = T == 3 ? 4 : 1;                    // rows requested together
     __shared__ __attribute__((aligned(16))) float buf[kNarrowRows * N * T > 1024 ? kNarrowRows * N * T : 1024];
     const int l = threadIdx.x & (L - 1), group = threadIdx.x / L, groups = 256 / L;
     const int quad = blockIdx.x * L + l;
@@ -711,8 +830,6 @@ __global__ void __launch_bounds__(256) wgrad_narrow_kernel(const float* __restri
     for (int k = 0; k < N; k++)
 #pragma unroll
         for (int j = 0; j < 4; j++) acc[k][j] = 0.f;
-    float column[4] = {0.f, 0.f, 0.f, 0.f};                   // of the wide operand; of the narrow one in column[0], its column ...
-    const int own_k = threadIdx.x & (kNarrow - 1), own_rows = threadIdx.x / kNarrow;      // ... and rows of this thread
     for (long r = r_lo; r < r_hi; r += kNarrowRows) {
         const int rows = r_hi - r < kNarrowRows ? (int)(r_hi - r) : kNarrowRows;
         __syncthreads();
@@ -722,8 +839,6 @@ __global__ void __launch_bounds__(256) wgrad_narrow_kernel(const float* __restri
             buf[row * (N * T) + (at - row * (n * T))] = narrow[r * n * T + at];
         }
         __syncthreads();
-        if (BIAS == kOfNarrow && blockIdx.x == 0 && own_k < n)
-            for (int row = own_rows; row < rows; row += 256 / kNarrow) column[0] += buf[row * N + own_k];
         for (int first = group; first < rows; first += kAhead * groups) {
             union { float4 v[T]; float f[4 * T]; } x[kAhead];
 #pragma unroll
@@ -744,9 +859,6 @@ __global__ void __launch_bounds__(256) wgrad_narrow_kernel(const float* __restri
                         for (int t = 0; t < T; t++)
 #pragma unroll
                             for (int j = 0; j < 4; j++) acc[k][j] = fmaf(b[k * T + t], x[u].f[j * T + t], acc[k][j]);
-                    if constexpr (BIAS == kOfWide)
-#pragma unroll
-                        for (int j = 0; j < 4; j++) column[j] += x[u].f[j];
                 }
             }
         }
@@ -769,17 +881,6 @@ __global__ void __launch_bounds__(256) wgrad_narrow_kernel(const float* __restri
 #pragma unroll
     for (int k = 0; k < N; k++)
         if (k < n) combine(k, acc[k]);                        // (uniform)
-    if constexpr (BIAS == kOfWide) combine(n, column);
-    if (BIAS == kOfNarrow && blockIdx.x == 0) {
-        __syncthreads();
-        buf[threadIdx.x] = column[0];
-        __syncthreads();
-        if (threadIdx.x < kNarrow) {
-            float s = buf[threadIdx.x];
-            for (int j = 1; j < 256 / kNarrow; j++) s += buf[kNarrow * j + threadIdx.x];
-            part[blockIdx.y * plane + (long)n * dim + threadIdx.x] = s;
-        }
-    }
 }
 
 // quad q of the plane (n, dim) to dW, transposed where x is the narrow operand, and those behind it to db (n_bias floats)
@@ -799,9 +900,10 @@ __global__ void __launch_bounds__(256) wgrad_narrow_reduce_kernel(const float4* 
     }
 }
 
-// lanes of a row, channel blocks, rows of a workgroup and their number: about four workgroups on each compute unit, of 64 rows at least
+// lanes of a row (plain rows: waves that share one, 64 channels each), channel blocks, rows of a workgroup and their number: about four
+// workgroups on each compute unit, of 64 rows at least
 struct NarrowPlan {
-    int lanes, blocks, n, dim;
+    int lanes, waves_c, blocks, n, dim;
     long rows, splits, plane;
 };
 NarrowPlan narrow_plan(long R, int dim_in, int dim_out) {
@@ -810,8 +912,9 @@ NarrowPlan narrow_plan(long R, int dim_in, int dim_out) {
     p.dim = dim_in < dim_out ? dim_out : dim_in;
     p.lanes = 16;
     while (p.lanes < 64 && 4 * p.lanes < p.dim) p.lanes *= 2;
+    p.waves_c = p.lanes / 16;
     p.blocks = (int)ceil_div(p.dim, 4 * p.lanes);
-    const long most = ceil_div(R, kNarrowRows), want = ceil_div(1024, p.blocks), s = want < most ? want : most;
+    const long most = ceil_div(R, kNarrowRows), want = 1024 / p.blocks, s = want < most ? want : most;   // (no more than are resident at once)
     p.rows = ceil_div(ceil_div(R, s < 1 ? 1 : s), kNarrowRows) * kNarrowRows;
     p.splits = ceil_div(R, p.rows);
     p.plane = (long)p.n * p.dim;
@@ -1065,17 +1168,18 @@ int mg_tensor_linear_wgrad_narrow(int inds, const float* dy, const float* x, lon
     if (db) p.plane += narrow_bias_floats(dim_in, dim_out);
     float* part = reinterpret_cast<float*>((reinterpret_cast<uintptr_t>(workspace) + 15) & ~uintptr_t(15));
     const dim3 grid((unsigned)p.blocks, (unsigned)p.splits);
-    const auto run = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, narrow, p.n, wide, p.dim, rows, p.rows, p.lanes, p.plane, part);
+    const auto run = [&](auto kernel, int across) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, narrow, p.n, wide, p.dim, rows, p.rows, across, p.plane, part);
     };
     const auto of_width = [&](auto width) {
         constexpr int N = decltype(width)::value;
-        if (inds == 0 && db) run(of_x ? wgrad_narrow_kernel<1, N, kOfWide> : wgrad_narrow_kernel<1, N, kOfNarrow>);
-        else if (inds == 0) run(wgrad_narrow_kernel<1, N>);
-        else if (inds == 1) run(wgrad_narrow_kernel<3, N>);
-        else if constexpr (N <= 5) run(wgrad_narrow_kernel<9, N>);
+        if (inds == 1) run(wgrad_narrow_kernel<3, N>, p.lanes);
+        else if constexpr (N <= 5) run(wgrad_narrow_kernel<9, N>, p.lanes);
     };
-    if (p.n <= 1) of_width(std::integral_constant<int, 1>{});
+    if (inds == 0)
+        run(db == nullptr ? wgrad_narrow_rows_kernel<kNoBias> : of_x ? wgrad_narrow_rows_kernel<kOfWide> : wgrad_narrow_rows_kernel<kOfNarrow>,
+            p.waves_c);
+    else if (p.n <= 1) of_width(std::integral_constant<int, 1>{});
     else if (p.n <= 2) of_width(std::integral_constant<int, 2>{});
     else if (p.n <= 4) of_width(std::integral_constant<int, 4>{});
     else if (p.n == 5) of_width(std::integral_constant<int, 5>{});
