@@ -462,11 +462,13 @@ def filters_of(blocks, x_a, x_v, r_ij_bond, r_ij):
     n = x_a.shape[2]
     none = [({}, {})] * len(blocks)
     messages = [m for b in blocks for m in (b._modules["message_bond"], b._modules["message"])]
-    if (any(diff.wants_grad(b, x_a, x_v, r_ij_bond, r_ij) for b in (blocks if torch.is_grad_enabled() else blocks[:1]))
-            or not all(diff.plain_call(m, Message) for m in messages)):
+    if any(diff.wants_grad(b, x_a, x_v, r_ij_bond, r_ij) for b in (blocks if torch.is_grad_enabled() else blocks[:1])):
         return none
     jobs, ahead = [], 0
     for k, m in enumerate(messages):
+        # (several blocks, and the first reads grids only: so do the others, as a rule, and looking at all seven of a model took 60 us)
+        if (k == 2 and not jobs) or not diff.plain_call(m, Message):
+            return none
         edges = (r_ij_bond, r_ij)[k % 2]
         E = edges.shape[0]
         params = None if m.keep_table else _plain_params(m.mlp_dist)
