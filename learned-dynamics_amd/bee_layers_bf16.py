@@ -36,10 +36,14 @@ def from_storage(s_a, s_v, s_d, batch):
             s_d.float().transpose(1, 2).reshape(batch, N, -1, 3, 3).contiguous())
 
 
-def _lin(W, x, comps):
-    """x (rows, comps, dim_in) or (rows, dim_in) bf16 -> same leading shape with dim_out."""
+def _lin(W, x, comps, onto=None):
+    """x (rows, comps, dim_in) or (rows, dim_in) bf16 -> same leading shape with dim_out; added to `onto`, which is overwritten, if given."""
     rows = x.shape[0]
-    y = ops.tensor_linear_bf16(W, x.reshape(rows * comps, x.shape[-1]))
+    x = x.reshape(rows * comps, x.shape[-1])
+    if onto is not None:
+        ops.tensor_linear_bf16(W, x, out=onto.view(rows * comps, W.shape[0]), accumulate=True)
+        return onto
+    y = ops.tensor_linear_bf16(W, x)
     return y if comps == 1 else y.reshape(rows, comps, -1)
 
 
@@ -104,9 +108,10 @@ def mlp_summed_over_rows(mlp, x, row_ptr, n_out, plus_identity=False, scale=1.0,
     return _mlp_after_sums(mlp, s_x, s_h, row_ptr, plus_identity, scale)
 
 
-def messages_forward(mod: Messages, graph: Graph, r_ij, s_a, s_v, s_d, node_order="cell", chain=True):
+def messages_forward(mod: Messages, graph: Graph, r_ij, s_a, s_v, s_d, node_order="cell", chain=True, onto=False):
     """Messages.forward (archs/diffuser_atoms15.py:238-253) on storage tensors; returns the three
-    0.1 * (sum over edges) increments in storage layout."""
+    0.1 * (sum over edges) increments in storage layout.  onto: added to s_a, s_v and s_d, of which the last two are
+    overwritten: their output linears add to them before the result is rounded."""
     if isinstance(node_order, str):
         node_order = getattr(graph, "cell_order", None)
     rows = s_a.shape[0]
@@ -132,9 +137,9 @@ def messages_forward(mod: Messages, graph: Graph, r_ij, s_a, s_v, s_d, node_orde
             psi_a, s_psi = ops.tensor_linear_bf16(Y0, P0.reshape(E, 3 * chan)), None
         B_a = mlp_summed_over_rows(mod.mlp_a, psi_a, graph.row_ptr, rows, plus_identity=True, scale=0.1,
                                    seg=graph.src32, s_x=s_psi)
-    B_v = _lin(_cat_Y(mod, LABELS_1, 0.1), S1.reshape(rows, 3, 5 * chan), 3)
-    B_d = _lin(_cat_Y(mod, LABELS_2, 0.1), S2.reshape(rows, 9, 5 * chan), 9)
-    return B_a, B_v, B_d
+    B_v = _lin(_cat_Y(mod, LABELS_1, 0.1), S1.reshape(rows, 3, 5 * chan), 3, s_v if onto else None)
+    B_d = _lin(_cat_Y(mod, LABELS_2, 0.1), S2.reshape(rows, 9, 5 * chan), 9, s_d if onto else None)
+    return (s_a + B_a if onto else B_a), B_v, B_d
 
 
 def _flat_gamma(gn):
@@ -175,8 +180,9 @@ def stack_forward(messages, prods, graph, r_ij, x_a, x_v, x_d, node_order="cell"
     inside the modules; float32 reference-layout tensors in and out."""
     batch = x_a.shape[0]
     s_a, s_v, s_d = to_storage(x_a, x_v, x_d)
+    if x_v.dtype == torch.bfloat16 or x_d.dtype == torch.bfloat16:       # (else to_storage has made tensors of its own)
+        s_v, s_d = s_v.clone(), s_d.clone()
     for msg, prod in zip(messages, prods):
-        d_a, d_v, d_d = messages_forward(msg, graph, r_ij, s_a, s_v, s_d, node_order=node_order)
-        s_a, s_v, s_d = s_a + d_a, s_v + d_v, s_d + d_d
+        s_a, s_v, s_d = messages_forward(msg, graph, r_ij, s_a, s_v, s_d, node_order=node_order, onto=True)
         s_a, s_v, s_d = self_tens_prods_forward(prod, s_a, s_v, s_d, batch, residual=True)
     return from_storage(s_a, s_v, s_d, batch)

@@ -59,6 +59,43 @@ def test_linear_bf16(ops, shape, y_bf16):
         torch.testing.assert_close(y2.cpu().double(), ref + x.double() @ W16.t(), rtol=1e-5, atol=4e-6 * dim_in ** 0.5)
 
 
+@pytest.mark.parametrize("rows,dim_in,dim_out,act", [(1, 640, 128, 0), (777, 640, 128, 0), (8193, 64, 256, 0), (300, 96, 96, 0),
+                                                     (1000, 32, 40, 0), (500, 128, 36, 0), (777, 64, 128, 2)])
+def test_linear_bf16_onto_bf16_rows(ops, rows, dim_in, dim_out, act):
+    """Added to bfloat16 rows before the one rounding of the result: whole pieces of 16 bytes, column tiles and rows cut short, and the
+    forms that keep the general epilogue (an activation, rows that are no whole pieces)."""
+    g = torch.Generator().manual_seed(rows + dim_out)
+    x, old = _bf(torch.randn(rows, dim_in, generator=g)), _bf(torch.randn(rows, dim_out, generator=g))
+    W = torch.randn(dim_out, dim_in, generator=g) / dim_in ** 0.5
+    hi = _bf(W).float()
+    pre = x.double() @ (hi + _bf(W - hi).float()).double().t()
+    y = old.cuda()
+    assert ops.tensor_linear_bf16(W.cuda(), x.cuda(), act=act, out=y, accumulate=True) is y
+    _close_bf16(y, old.double() + (torch.where(pre > 0, pre, 0.1 * pre) if act == 2 else pre))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_stack_bf16_keeps_its_inputs(pkg, dtype):
+    """The messages add to the features in place: to tensors of the stack's own, also where the inputs are bfloat16 and lie as the
+    storage does (one channel)."""
+    b16, bl = (importlib.import_module(f"learned-dynamics_amd.{m}") for m in ("bee_layers_bf16", "bee_layers"))
+    x_a, x_v, x_d = torch.randn(2, 5, 32).to(dtype), torch.randn(2, 5, 1, 3).to(dtype), torch.randn(2, 5, 1, 3, 3).to(dtype)
+    kept, seen = [t.clone() for t in (x_a, x_v, x_d)], []
+
+    def messages(mod, graph, r_ij, s_a, s_v, s_d, node_order, onto):
+        assert onto
+        seen.append([t.clone() for t in (s_a, s_v, s_d)])
+        return s_a + 1, s_v.add_(1), s_d.add_(1)
+    real = b16.messages_forward, b16.self_tens_prods_forward
+    b16.messages_forward, b16.self_tens_prods_forward = messages, lambda mod, a, v, d, batch, residual: (a, v, d)
+    try:
+        out = b16.stack_forward([None, None], [None, None], None, None, x_a, x_v, x_d)
+    finally:
+        b16.messages_forward, b16.self_tens_prods_forward = real
+    assert all(torch.equal(a, b) for a, b in zip((x_a, x_v, x_d), kept))
+    assert len(seen) == 2 and all(o.shape == k.shape and o.dtype == torch.float32 for o, k in zip(out, kept))
+
+
 def test_linear_bf16_errors(ops):
     W = torch.randn(64, 48, device="cuda")
     with pytest.raises(RuntimeError, match="multiple of 32"):
