@@ -83,32 +83,6 @@ def test_tensor_linear_and_its_derivatives(ext, inds):
         ext.tensor_linear(0, W.cuda(), torch.randn(24, 3, device="cuda").t())
 
 
-def test_tensor_linear_without_a_record(ext):
-    """Nothing to record: the same values with and without gradients enabled.  What the function does not support is refused on
-    this path as on the recorded one: tangents, vmap, transforms."""
-    import torch.autograd.forward_ad as fwAD
-    g = torch.Generator().manual_seed(29)
-    W, x = torch.randn(40, 24, generator=g).cuda(), torch.randn(13, 24, generator=g).cuda()
-    Wg = W.clone().requires_grad_()
-    recorded = ext.tensor_linear(0, Wg, x)
-    assert recorded.requires_grad and not ext.tensor_linear(0, W, x).requires_grad
-    with torch.no_grad():
-        plain = ext.tensor_linear(0, Wg, x)
-    with torch.inference_mode():
-        inference = ext.tensor_linear(0, Wg, x)
-    assert not plain.requires_grad and torch.equal(plain, recorded) and torch.equal(inference, plain)
-    for context in (torch.enable_grad, torch.no_grad):
-        with context(), fwAD.dual_level():
-            with pytest.raises(RuntimeError):
-                ext.tensor_linear(0, W, fwAD.make_dual(x, torch.ones_like(x)))
-        with context(), pytest.raises(RuntimeError):
-            torch.func.vmap(lambda t: ext.tensor_linear(0, W, t))(x)
-        with context(), pytest.raises(RuntimeError):
-            torch.func.jvp(lambda t: ext.tensor_linear(0, W, t), (x,), (torch.ones_like(x),))
-        with context(), pytest.raises(RuntimeError):
-            torch.func.grad(lambda t: ext.tensor_linear(0, W, t).sum())(x)
-
-
 def test_bee_and_cow_equal_the_ctypes_route(ext, ops):
     g = torch.Generator().manual_seed(9)
     rows, chan = 77, 33
@@ -262,3 +236,29 @@ def test_other_threads_run_while_the_norms_are_read_back(ops):
     if ended - began < 0.05:
         pytest.skip("the device was not busy long enough")
     assert sum(began < t < ended for t in stamps) > 10
+
+
+def test_tensor_linear_without_a_record(ext):
+    """Nothing to record: the same values with and without gradients enabled.  What the function does not support is refused on
+    this path as on the recorded one: tangents, vmap, transforms."""
+    import torch.autograd.forward_ad as fwAD
+    g = torch.Generator().manual_seed(29)
+    W, x = torch.randn(40, 24, generator=g).cuda(), torch.randn(13, 24, generator=g).cuda()
+    Wg = W.clone().requires_grad_()
+    recorded = ext.tensor_linear(0, Wg, x)
+    assert recorded.requires_grad and not ext.tensor_linear(0, W, x).requires_grad
+    with torch.no_grad():
+        plain = ext.tensor_linear(0, Wg, x)
+    with torch.inference_mode():
+        inference = ext.tensor_linear(0, Wg, x)
+    assert not plain.requires_grad and torch.equal(plain, recorded) and torch.equal(inference, plain)
+    for context in (torch.enable_grad, torch.no_grad):
+        with context(), fwAD.dual_level():
+            with pytest.raises(RuntimeError):
+                ext.tensor_linear(0, W, fwAD.make_dual(x, torch.ones_like(x)))
+        with context(), pytest.raises(RuntimeError):
+            torch.func.vmap(lambda t: ext.tensor_linear(0, W, t))(x)
+        with context(), pytest.raises(RuntimeError):
+            torch.func.jvp(lambda t: ext.tensor_linear(0, W, t), (x,), (torch.ones_like(x),))
+        with context(), pytest.raises(RuntimeError):
+            torch.func.grad(lambda t: ext.tensor_linear(0, W, t).sum())(x)
