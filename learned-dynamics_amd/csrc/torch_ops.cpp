@@ -407,6 +407,10 @@ std::tuple<at::Tensor, OptTensor> linear_fwd(int64_t inds, const at::Tensor& W, 
             b = Bound{row_bound, (float)mul, (float)add, rows_per};
             TORCH_CHECK(row_bound->dim() == 2 && (row_bound->size(0) * rows_per == R || row_bound->size(0) == 1),
                         "row_bound must be (rows / rows_per_bound, parts)");
+        } else {
+            // (a pass of its own: the binding's fp32 linear is to stay the cheaper call for small plain rows, 5.7 us of host time at
+            // 256 x 64 -> 64 in a process of many streams where this operator takes 5.2 without the pass; chains find theirs on the way)
+            b = Bound{row_absmax(x.reshape({R, dim_in}))};
         }
         run_f16x2(W, dim_in, fp(x), R, b, bias, act, accumulate, out_comps, y, rowmax_buffer(dim_in), sequential);
     } else if (mode == kModeBf16x3 && plain_rows && dim_in % 32 == 0 && dim_in >= 64 && dim_out >= 64 && R >= 1024 &&
