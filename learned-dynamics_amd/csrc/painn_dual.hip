@@ -292,14 +292,19 @@ __device__ __forceinline__ void st_unless_null(float* p, long off, const T& r) {
         for (int q = 0; q < V; q += 2) *reinterpret_cast<float2*>(p + off + q) = make_float2(r.f[q], r.f[q + 1]);
     }
 }
+// a + b with a rounded as it would be where it is stored: contracted into the product that a may be, x + q w moved a layer's results
+// by a spacing of the sum, and with them the positions that a step subtracts from the old ones (an instruction more: the kernels wait
+// for memory)
 template <int V>
 __device__ __forceinline__ Chans<V> plus(Chans<V> a, const Chans<V>& b) {
+#pragma clang fp contract(off)
 #pragma unroll
     for (int j = 0; j < V; j++) a.f[j] += b.f[j];
     return a;
 }
 template <int V>
 __device__ __forceinline__ Vec3s<V> plus(Vec3s<V> a, const Vec3s<V>& b) {
+#pragma clang fp contract(off)
 #pragma unroll
     for (int j = 0; j < 3 * V; j++) a.f[j] += b.f[j];
     return a;

@@ -53,6 +53,36 @@ def test_se3ito_forward_against_oracle(pkg, mutate_pos):
         assert not bool(v[1].any())            # (s, t) = (0, 1) with positions left in place: identically zero
 
 
+@pytest.mark.parametrize("n, N", [(64, 150), (128, 371)])
+def test_a_step_that_moves_positions_rounds_its_additions(pkg, monkeypatch, n, N):
+    """Value and derivative of a mutate_pos step with the layers' inputs added inside their kernels against additions of their own:
+    the same bits.  The output subtracts moved positions from the old ones, so that one rounding less in the layer below is whole
+    spacings of the positions in it."""
+    diff = importlib.import_module("learned-dynamics_amd.differentiable")
+    mp, model, _ = _model(n, N, (1, 2), 5.0, True, seed=0x947 + n)
+    x0, one_hot, bs, bd = _system(1, N, 25.0, seed=5)
+    x0 = x0.cuda()
+    z, v = x0 + 0.3 * torch.randn_like(x0), torch.randn_like(x0)
+    topo = mp.Topology(one_hot.cuda(), bs.cuda(), bd.cuda())
+    s, t = torch.zeros(1).cuda(), torch.full((1,), 0.02).cuda()
+
+    def step():
+        return [o.detach() for o in diff.jvp(lambda z, t: model((s, t), x0, z, (40.0,) * 3, topo), (z, t), (v, torch.ones_like(t)))]
+
+    inside, calls = step(), []
+    for name in ("painn_message", "painn_update"):
+        def outside(layer, *args, residual=False, own=getattr(diff, name)):
+            calls.append(layer)
+            args, residual = (args[:-1], args[-1]) if isinstance(args[-1], bool) else (args, residual)
+            x_a, x_v = [a for a in args if torch.is_tensor(a)][:2]
+            out = own(layer, *args)
+            return tuple(diff.add(x, d) for x, d in zip((x_a, x_v), out)) if residual else out
+        monkeypatch.setattr(diff, name, outside)
+    for a, b in zip(inside, step()):
+        assert torch.equal(a, b), float((a - b).norm() / b.norm())
+    assert len(calls) == 9
+
+
 @pytest.mark.parametrize("n, N, B", [(64, 150, 1), (128, 130, 2), (128, 400, 8)])
 def test_filters_of_all_blocks_together(pkg, n, N, B):
     """A stack whose blocks' filters (of every edge, of grids, of some of both) are evaluated ahead against its blocks called one by one
