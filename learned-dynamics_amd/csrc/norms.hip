@@ -117,6 +117,13 @@ __device__ __forceinline__ void update_vec(const UpdateVec& a, long r, int n, in
     a.out_v[t] = o0; a.out_v[t + 1] = o1; a.out_v[t + 2] = o2;
 }
 
+// (y + first) + second, each rounded: neither is contracted into the product that y is, nor are they added to each other first
+__device__ __forceinline__ float added(float y, float first, float second) {
+#pragma clang fp contract(off)
+    y += first;
+    return y + second;
+}
+
 // mode 0 (TensGroupNorm): y = gamma[c] * v / sqrt(eps + mean(sum_comp v^2))
 // mode 1 (ScalGroupNorm, T = 1): y = beta[c] + gamma[c] * (v - mean) / sqrt(eps + var)
 // then y += add (optional, add_stride) and y += res (optional, same layout as out).
@@ -142,7 +149,7 @@ __global__ void __launch_bounds__(256) group_apply_kernel(const float* __restric
     const bool live = k < CT;
     const long x_row = x_stride * T, m_row = mul_stride * T, a_row = add_stride * T;
     constexpr int kAhead = 4;                                      // nodes at a time; the first ones are on their way during the fold
-    float v[kAhead], plus[kAhead];
+    float v[kAhead], first[kAhead], second[kAhead];                // value, what is added
     auto fetch = [&](int i) {
 #pragma unroll
         for (int u = 0; u < kAhead; u++) {
@@ -150,8 +157,8 @@ __global__ void __launch_bounds__(256) group_apply_kernel(const float* __restric
             const long row = (long)b * N + (node < N ? node : N - 1);
             v[u] = live ? x[row * x_row + k] : 0.f;
             if (mul && live) v[u] *= mul[row * m_row + k];
-            plus[u] = add && live ? add[row * a_row + k] : 0.f;
-            if (res && live) plus[u] += res[row * CT + k];
+            first[u] = add && live ? add[row * a_row + k] : 0.f;
+            second[u] = res && live ? res[row * CT + k] : 0.f;
         }
     };
     fetch(blockIdx.y);
@@ -170,7 +177,7 @@ __global__ void __launch_bounds__(256) group_apply_kernel(const float* __restric
         for (int u = 0; u < kAhead; u++) {
             const int node = i + u * (int)gridDim.y;
             const float y = mode == 0 ? ga * (v[u] / denom) : be + ga * ((v[u] - mean) / denom);
-            if (node < N) out[((long)b * N + node) * CT + k] = y + plus[u];
+            if (node < N) out[((long)b * N + node) * CT + k] = added(y, first[u], second[u]);
             if constexpr (VEC != 0)
                 if (node < N) update_vec<VEC - 1>(vec, (long)b * N + node, CT, k);
         }

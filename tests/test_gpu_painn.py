@@ -797,3 +797,16 @@ def test_group_norm_and_vector_output_in_one_pass(ops, batch, nodes, n, groups, 
         L.check(lib.mg_painn_update_post(p(lrv), layout, p(ip), p(y), batch, nodes, n, groups, 1.0, p(gamma), p(beta), res_a, res_v,
                                          p(scratch), p(out[2]), p(out[3]), stream))
         assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[3])
+
+
+@pytest.mark.parametrize("mode, nodes, comps", [(1, 1, 1), (1, 337, 1), (1, 2051, 1), (0, 337, 3), (0, 70, 9)])
+def test_group_norm_adds_its_operands_one_after_the_other(ops, mode, nodes, comps):
+    """(norm + add) + res, each sum rounded: the bits of additions outside the kernel."""
+    g = torch.Generator().manual_seed(nodes + comps)
+    shape = (2, nodes, 64) + {1: (), 3: (3,), 9: (3, 3)}[comps]
+    x, add, res = (torch.randn(*shape, generator=g).cuda() for _ in range(3))
+    gamma, beta = torch.randn(64, generator=g).cuda(), torch.randn(64, generator=g).cuda() if mode else None
+    plain = ops.group_norm(mode, x, 4, gamma, beta)
+    for a, r in ((None, res), (add, None), (add, res)):
+        want = plain if a is None else plain + a
+        assert torch.equal(ops.group_norm(mode, x, 4, gamma, beta, add=a, res=r), want if r is None else want + r)
