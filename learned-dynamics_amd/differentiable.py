@@ -920,7 +920,8 @@ def painn_message(msg, graph, x_a, x_v, r_ij, residual=False):
     actv = _mlp_silu_pair(msg.mlp_actv, x_a)
     rows = _filter_grid_rows(msg, r_ij)
     n = x_v.size(-2)
-    if (rows and n % 4 == 0 and ops.painn_combine_supported(n) and not any(has_tangent(t) for t in (x_a, x_v))
+    # (actv has a tangent without x_a where its MLP's weights have one)
+    if (rows and n % 4 == 0 and ops.painn_combine_supported(n) and actv[1] is None and not any(has_tangent(t) for t in (x_a, x_v))
             and r_ij.is_contiguous() and not getattr(graph, "padded", False)):
         table = mlp_silu(msg.mlp_dist, msg._grid_encoding(rows, 0.0, r_ij.device))
         flat_v, flat_a = gl._flat_nodes(graph, x_v), gl._flat_nodes(graph, x_a) if residual else None

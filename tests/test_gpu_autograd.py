@@ -8,6 +8,7 @@ import importlib
 
 import pytest
 import torch
+import torch.autograd.forward_ad as fwAD
 
 from oracle import layers as OL
 from oracle import models as OM
@@ -1562,3 +1563,32 @@ def test_layers_that_add_their_input(pkg, E, n):
             if a is not None:
                 err, size = float((a.detach() - b.detach()).norm()), float(a.detach().norm())
                 assert err <= 2e-6 * size, (k, err, size)
+
+
+@pytest.mark.parametrize("residual", [False, True])
+def test_message_with_tangents_on_the_weights_of_its_node_mlp(pkg, residual):
+    """Forward mode over mlp_actv's weights alone, the inputs without tangents, on as many edges as the filter is read from its grid
+    for: the derivative that the message with the filter MLP on every edge gives, not none."""
+    painn = importlib.import_module("learned-dynamics_amd.painn")
+    gl = importlib.import_module("learned-dynamics_amd.graph_layers")
+    g = torch.Generator().manual_seed(0x947)
+    torch.manual_seed(0x947)
+    N, E, n = 300, 30000, 64
+    src = torch.sort(torch.randint(0, N, (E,), generator=g)).values
+    graph = gl.Graph(src.cuda(), torch.randint(0, N, (E,), generator=g).cuda(), None, 1, N)
+    msg = painn.Message(5.0, n).cuda()
+    assert 0 < msg.table_rows() <= E // 4
+    r, x_a, x_v = (torch.randn(*s, generator=g).cuda() for s in ((E, 3), (1, N, n), (1, N, n, 3)))
+    names = [f"mlp_actv.layers.{k}.{w}" for k in (0, 4) for w in ("weight", "bias")]
+    params = dict(msg.named_parameters())
+    tangents = {k: torch.randn(params[k].shape, generator=g).cuda() for k in names}
+    ways = []
+    for msg.use_table in (True, False):
+        with fwAD.dual_level():
+            duals = {k: fwAD.make_dual(params[k], t) for k, t in tangents.items()}
+            out = torch.func.functional_call(msg, duals, (graph, x_a, x_v, r), dict(residual=residual))
+            ways.append([fwAD.unpack_dual(o) for o in out])
+    for (p, t), (p_ref, t_ref) in zip(*ways):
+        assert t is not None and t_ref is not None and float(t_ref.detach().norm()) > 0
+        for a, b in ((p, p_ref), (t, t_ref)):
+            assert float((a - b).detach().norm()) <= 1e-5 * float(b.detach().norm())
