@@ -81,6 +81,18 @@ def _mlp_params(mlp):
     return weights, biases
 
 
+def _own_parameters(mlp):
+    """The parameters that an MLP's filter depends on, to be stamped: out of the modules' dictionaries where the three linears are
+    plain and hold theirs (a walk over the modules is 15 us), else whatever parameters() finds.  A weight that is computed at every
+    access (torch.nn.utils.parametrize) is a new tensor each time, often at the address of the one before: no stamp tells two
+    of them apart, those of the parameters that it is computed from do."""
+    if type(mlp) is MLP:
+        linears = list(mlp._modules["layers"]._modules.values())[0:5:2]
+        if all(type(lin) is nn.Linear and {"weight", "bias"} <= lin._parameters.keys() for lin in linears):
+            return [p for lin in linears for p in (lin._parameters["weight"], lin._parameters["bias"]) if p is not None]
+    return list(mlp.parameters())
+
+
 def _plain_params(mlp):
     """_mlp_params of a submodule whose call may be replaced by one that reads its parameters, else None."""
     return _mlp_params(mlp) if diff.plain_call(mlp, MLP) else None
@@ -349,9 +361,7 @@ class Message(nn.Module):
         for TABLE_RECHECK changes of the weights before it is made again: one optimizer step moves the
         interpolation error by far less than the factor ten between TABLE_ATOL / TABLE_RTOL and the layer
         tolerance, and the check costs host synchronisations that a training step should not pay every time."""
-        params = _mlp_params(self.mlp_dist) if type(self.mlp_dist) is MLP else None
-        # (a walk over the modules is 15 us)
-        stamp = ops.stamp(self.mlp_dist.parameters() if params is None else [*params[0], *params[1]], keep_unversioned=True)
+        stamp = ops.stamp(_own_parameters(self.mlp_dist), keep_unversioned=True)
         cache = self.__dict__.setdefault("_table_cache", {})
         if cache.get("stamp") != stamp:
             training = diff.wants_grad(self.mlp_dist)
