@@ -972,15 +972,28 @@ def tensor_version(t):
     return -1 if t.is_inference() else (_cache_epoch << 40) | t._version
 
 
+class _Stamp(tuple):
+    """Compares as the tuple it is; held: tensors that are not to go while something carries this stamp."""
+
+
 def stamp(tensors, keep_unversioned=False):
-    """What a cache of something computed from these tensors compares: objects, versions, addresses.  With an inference
+    """What a cache of something computed from these tensors compares: objects, versions, addresses.  A tensor that is no
+    parameter may be gone after the call (a weight computed at every access): its memory is held as long as the stamp, so that no
+    later one has its address.  With an inference
     tensor among them (no version counter) the stamp equals no other, so the cached value is rebuilt; with
     keep_unversioned such a tensor is stamped by object, address and the epoch of invalidate_weight_caches instead
     (for decisions that are expensive to re-make and that a caller who writes such tensors in place can reset)."""
+    tensors = tuple(tensors)
     st = tuple((id(t), tensor_version(t), t.data_ptr()) for t in tensors)
-    if all(v[1] >= 0 for v in st):
-        return st
-    return tuple((i, v if v >= 0 else -1 - _cache_epoch, p) for i, v, p in st) if keep_unversioned else (object(),)
+    if not all(v[1] >= 0 for v in st):
+        if not keep_unversioned:
+            return (object(),)
+        st = tuple((i, v if v >= 0 else -1 - _cache_epoch, p) for i, v, p in st)
+    passing = [t.detach() for t in tensors if not isinstance(t, torch.nn.Parameter)]
+    if passing:
+        st = _Stamp(st)
+        st.held = passing
+    return st
 
 
 @contextlib.contextmanager

@@ -1,5 +1,5 @@
-"""When the decision for a filter grid is made again (learned-dynamics_amd/painn.py, Message.table_rows): host logic, the error of a
-grid stubbed, so that no kernel of the library runs."""
+"""When what is kept of weights is made again: the decision for a filter grid (learned-dynamics_amd/painn.py, Message.table_rows, with
+the error of a grid stubbed) and the stamps that caches compare (ops.stamp).  Host logic, no kernel of the library runs."""
 import importlib
 
 import pytest
@@ -39,3 +39,22 @@ def test_changed_weights_are_decided_on_again(changed):
         msg.table_rows()
         msg.table_rows()
         assert len(decisions) == k
+
+
+def test_a_weight_computed_at_every_access_is_never_taken_for_the_one_before(ops):
+    """The stamp of what is kept of such a weight: another one after a change of what it is computed from, although the allocator
+    hands the address out again; that of a parameter or of a tensor that stays is the same until it is written."""
+    lin = torch.nn.Linear(64, 64)
+    stays = torch.randn(8, 8)
+    kept = ops.stamp((lin.weight, stays))
+    assert ops.stamp((lin.weight, stays)) == kept
+    stays.add_(1.0)
+    assert ops.stamp((lin.weight, stays)) != kept
+    torch.nn.utils.parametrize.register_parametrization(lin, "weight", _Scaled())
+    with torch.no_grad():
+        kept = [ops.stamp((lin.weight, lin.bias))]
+        for _ in range(20):
+            lin.parametrizations.weight.original.mul_(3.0)
+            kept.append(ops.stamp((lin.weight, lin.bias)))
+            assert kept[-1] != kept[-2]
+            del kept[0]
