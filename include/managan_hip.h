@@ -741,7 +741,8 @@ int mg_painn_grid_rows_by_node(const float* r_ij, long n_edges, const int* row_p
 int mg_painn_grid_table_grad(const int* order, const int* bucket_ptr, const int* src, const int* dst, int n_nodes, long n_edges,
                              const float* r_ij, int table_rows, float period, float epsilon, const float* g_v, const float* g_a,
                              const float* actv_sliced, const float* v, int n, void* workspace, float* d_table, mg_stream_t stream);
-/* order: the positions of keys (0 .. key_limit - 1) in the order of a stable sort; sorted_keys: the keys in that order. */
+/* order: the positions of keys (0 .. key_limit - 1) in the order of a stable sort; sorted_keys: the keys in that order.  A workspace of
+ * the bytes of one count serves every smaller one. */
 int mg_sort_by_key_workspace_bytes(long count, size_t* bytes /* host */);
 int mg_sort_by_key(const int* keys, long count, int key_limit, void* workspace, int* order, int* sorted_keys, mg_stream_t stream);
 /* the same with `order` the values that go with the keys (NULL: their positions) */

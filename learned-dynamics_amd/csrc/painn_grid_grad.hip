@@ -11,6 +11,7 @@
 // edges).  16384 nodes, 1.6 M edges, n = 128: see the figures at the two kernels.
 #include "common.hpp"
 #include "lane_sums.hpp"
+#include <algorithm>
 
 namespace mg {
 namespace {
@@ -568,7 +569,10 @@ int mg_painn_grid_table_grad(const int* order, const int* bucket_ptr, const int*
 
 int mg_sort_by_key_workspace_bytes(long count, size_t* bytes) {
     MG_REQUIRE(bytes && count >= 0, "mg_sort_by_key_workspace_bytes: bad argument");
-    *bytes = ((size_t)(ceil_div(count, 256L * sort_per_thread(count)) + 1) * kDigits + 3 * (size_t)count) * sizeof(int);
+    // (up to 256 chunks of every length but the longest: a smaller count may have more chunks than this one)
+    const long own = ceil_div(count, 256L * sort_per_thread(count)), shortest = ceil_div(count, 256L * 2);
+    const long chunks = std::max(own, std::min(256L, shortest));
+    *bytes = ((size_t)(chunks + 1) * kDigits + 3 * (size_t)count) * sizeof(int);
     return MG_OK;
 }
 

@@ -47,6 +47,20 @@ def test_host_only_entry_points():
     assert lib.mg_status_string(0) == b"ok"
 
 
+def test_a_sort_workspace_serves_every_smaller_count():
+    """Chunks grow with the count, so that one more element may need fewer of them: what is asked for never falls, and covers a count's
+    own chunks (512 counts each, one row of totals, spare keys and values and the positions between passes)."""
+    lib = importlib.import_module("learned-dynamics_amd._lib").load()
+    size, before = ctypes.c_size_t(0), 0
+    edges = [512 * 2 ** k + d for k in range(13) for d in (-1, 0, 1)] + [4096 * 300 + d for d in (-1, 0, 1)]
+    for count in sorted({0, 1, 2, 511, *edges, *range(1000, 1400000, 7919)}):
+        assert lib.mg_sort_by_key_workspace_bytes(count, ctypes.byref(size)) == 0
+        per = next(p for p in (2, 4, 8, 16) if p == 16 or count <= 65536 * p)
+        chunks = -(-count // (256 * per))
+        assert size.value >= max(before, 4 * ((chunks + 1) * 512 + 3 * count)), count
+        before = size.value
+
+
 def test_shims_expose_reference_symbols():
     pkg = importlib.import_module("learned-dynamics_amd")
     pkg.install_shims()

@@ -1513,6 +1513,24 @@ def test_sort_by_key_in_chunks_of_every_length(ops, count):
         assert torch.equal(order.cpu().long(), want.indices) and torch.equal(ordered.cpu(), want.values), limit
 
 
+@pytest.mark.parametrize("count, sized_for", [(2 ** 17, 2 ** 17 + 1), (2 ** 18, 2 ** 18 + 1), (2 ** 19, 2 ** 19 + 1), (513, 100000)])
+def test_sort_by_key_in_the_workspace_of_a_larger_count(ops, count, sized_for):
+    """More chunks than the count that the workspace was sized for has: nothing behind it is written."""
+    import ctypes
+    L = importlib.import_module("learned-dynamics_amd._lib")
+    lib, size = L.load(), ctypes.c_size_t(0)
+    L.check(lib.mg_sort_by_key_workspace_bytes(sized_for, ctypes.byref(size)))
+    keys = torch.randint(0, 2 ** 18, (count,), generator=torch.Generator().manual_seed(count), dtype=torch.int32)
+    on_device, workspace = keys.cuda(), torch.full((size.value // 4 + 2 ** 18,), -7, dtype=torch.int32, device="cuda")
+    order, ordered = torch.empty_like(on_device), torch.empty_like(on_device)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    L.check(lib.mg_sort_by_key(p(on_device), count, 2 ** 18, p(workspace), p(order), p(ordered),
+                               ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    want = torch.sort(keys, stable=True)
+    assert torch.equal(order.cpu().long(), want.indices) and torch.equal(ordered.cpu(), want.values)
+    assert bool((workspace[size.value // 4:] == -7).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
 def test_row_pointers_of_long_runs_of_empty_rows(ops, dtype):
     """Runs of rows without an edge, before, between and behind the rows that have one, in one wave of edges and across waves."""
