@@ -158,15 +158,19 @@ __device__ __forceinline__ void put_row(__amdgpu_buffer_rsrc_t r, unsigned lane_
     __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), r, (int)lane_bytes, (int)row_bytes, 2);
 }
 
-// The running sums of one (node, channel).  phi rh is formed once per edge and multiplies l directly; the sums 022 are symmetric and
-// 111 is the antisymmetric part of 112, so 54 values and 93 multiply-adds an edge make the 60 sums and the three products (they
-// took 122 with every product formed by itself).
+// The running sums of one (node, channel).  phi rh is formed once per edge and multiplies l directly, and the sums 022 are symmetric:
+// 57 values and 112 multiply-adds an edge make the 60 sums and the three products (122 with every product formed by itself).
+// Where features lie along the edges or across them, cross and scalar products cancel: these are formed of l and rh, whose
+// products cancel to a rounding of their own, before phi multiplies them.  (Taken apart further they lose what is left: 111 as the
+// antisymmetric part of the sum 112 was 2.8 times as far from float64 at 16 neighbours along the edges and 4.2 times at 90, 212 out
+// of l and phi rh, its two products added one after the other, 1.3 to 1.8 times on any features, 110 and 121 out of l . phi rh 1.5
+// times across the edges; 93 multiply-adds with all three.)
 struct NodeSums {
-    float v011[3], v101[3], v121[3], v211[3], d022[6], d202[9], d112[9], d222[9], d212[9];
+    float v011[3], v101[3], v121[3], v211[3], v111[3], d022[6], d202[9], d112[9], d222[9], d212[9];
     static __device__ __forceinline__ constexpr int sym(int x, int y) { return x <= y ? x * (5 - x) / 2 + y : y * (5 - y) / 2 + x; }
     __device__ __forceinline__ void clear() {
 #pragma unroll
-        for (int x = 0; x < 3; x++) v011[x] = v101[x] = v121[x] = v211[x] = 0.f;
+        for (int x = 0; x < 3; x++) v011[x] = v101[x] = v121[x] = v211[x] = v111[x] = 0.f;
 #pragma unroll
         for (int k = 0; k < 6; k++) d022[k] = 0.f;
 #pragma unroll
@@ -181,8 +185,9 @@ struct NodeSums {
             pr[x] = phi * rh[x];
             t[x] = l2[3 * x] * rh[0] + l2[3 * x + 1] * rh[1] + l2[3 * x + 2] * rh[2];
         }
+        auto cross = [&](const float* v, int x) { return v[(x + 1) % 3] * rh[(x + 2) % 3] - v[(x + 2) % 3] * rh[(x + 1) % 3]; };
         p0[0] = phi * l[0];
-        p0[1] = l1[0] * pr[0] + l1[1] * pr[1] + l1[2] * pr[2];
+        p0[1] = phi * (l1[0] * rh[0] + l1[1] * rh[1] + l1[2] * rh[2]);
         p0[2] = t[0] * pr[0] + t[1] * pr[1] + t[2] * pr[2];
 #pragma unroll
         for (int x = 0; x < 3; x++) {
@@ -191,15 +196,15 @@ struct NodeSums {
             v101[x] += phi * l1[x];
             v121[x] += p0[1] * rh[x];
             v211[x] += phi * t[x];
+            v111[x] += phi * cross(l1, x);
 #pragma unroll
             for (int y = 0; y < 3; y++) {
-                const int k = 3 * x + y, a = 3 * x + (y + 1) % 3, b = 3 * x + (y + 2) % 3;
+                const int k = 3 * x + y;
                 if (y >= x) d022[sym(x, y)] += plx * rh[y];
                 d202[k] += phi * l2[k];
                 d112[k] += l1[x] * pr[y];
                 d222[k] += t[x] * pr[y];
-                d212[k] += l2[a] * pr[(y + 2) % 3];                                     // (L[x,:] x phi rh)[y]
-                d212[k] -= l2[b] * pr[(y + 1) % 3];
+                d212[k] += phi * cross(l2 + 3 * x, y);
             }
         }
     }
@@ -207,12 +212,11 @@ struct NodeSums {
     __device__ __forceinline__ void rows(float (&s1)[15], float (&s2)[45]) const {
 #pragma unroll
         for (int x = 0; x < 3; x++) {
-            const int a = (x + 1) % 3, b = (x + 2) % 3;
             s1[x * 5] = v011[x];
             s1[x * 5 + 1] = v101[x];
             s1[x * 5 + 2] = v121[x];
             s1[x * 5 + 3] = v211[x];
-            s1[x * 5 + 4] = d112[3 * a + b] - d112[3 * b + a];
+            s1[x * 5 + 4] = v111[x];
 #pragma unroll
             for (int y = 0; y < 3; y++) {
                 const int k = 3 * x + y;
@@ -375,11 +379,12 @@ bee_message_kernel(const MessageArgs<T> g) {
 // no registers wait for them.  The compiler waits for every such load before any read of LDS, so they are written out and
 // counted here: a load reads its address registers when it issues and has no destination registers, nothing depends on it
 // but the wave's own slice of LDS.
-// Against operands one edge ahead in registers and 122 multiply-adds an edge (bee_message_kernel before NodeSums): 65 536 nodes with 90
-// neighbours, 128 channels of bf16, 3.28 -> 2.72 ms; 32 x 2048 with 16, 256 channels of float with the rank-2 linear, 2.19 -> 2.04 ms;
-// 2048 nodes of it 84 -> 73 us.  Three edges ahead take 2.94 ms, 2.07 ms and 78 us, two chunks a wave (two waves a SIMD) 3.34 ms,
-// 2.18 ms and 85 us.  What bounds it: bf16 by vector issue (109 instructions an edge, 0.9 of the cycles at the 2.0 GHz that the power
-// leaves); float by what it stores and gathers (without the stores of P0 1.61 ms, with every gather a hit 1.76).
+// Against operands one edge ahead in registers and 122 multiply-adds an edge (bee_message_kernel before NodeSums), both in turn on
+// one machine: 65 536 nodes with 90 neighbours, 128 channels of bf16, 3.22 -> 2.77 ms; 32 x 2048 with 16, 256 channels of float with
+// the rank-2 linear, 2.11 -> 2.02 ms; 2048 nodes of it 87 -> 80 us.  With 93 multiply-adds an edge it was 2.66 ms, 1.99 ms and 76 us,
+// three edges ahead 2.94 ms, 2.07 ms and 78 us, two chunks a wave (two waves a SIMD) 3.34 ms, 2.18 ms and 85 us.  What bounds it:
+// bf16 vector issue (128 vector instructions an edge; with 109 of them 0.9 of the cycles at the 2.0 GHz that the power leaves);
+// float what it stores and gathers (without the stores of P0 1.61 of 2.04 ms, with every gather a hit 1.76).
 constexpr int kDepth = 2;
 typedef int intx4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ intx4 row_words(const void* base, long bytes) {

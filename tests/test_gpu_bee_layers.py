@@ -177,6 +177,82 @@ def test_bee_message_rows_of_every_short_length(ops, chan, bf16):
                 assert float((S[:, :, k] - ref).abs().max()) <= 1e-5 * float(ref.abs().max()), lab
 
 
+@pytest.mark.parametrize("features", ["any", "along", "across"])
+@pytest.mark.parametrize("neighbours", [16, 90])
+def test_bee_message_is_as_exact_as_products_formed_one_by_one(ops, neighbours, features):
+    """Sums over edges and scalar products against float64, beside those of every product formed by itself in fp32 with fused
+    multiply-adds, edge after edge: no farther off, also where the features lie along their edges or across them and the cross or
+    the scalar products cancel.  Root mean squares over 24 nodes x 64 channels x components, whose own spread is some 2 %: 1.1 times."""
+    g = torch.Generator().manual_seed(neighbours)
+    N, chan = 24, 64
+    E = N * neighbours                                                   # (an edge's features are its own: node e is its destination)
+    unit = torch.randn(E, 3, generator=g, dtype=torch.float64)
+    unit /= unit.norm(dim=1, keepdim=True)
+    rh = unit.float()
+    l0, l1, l2 = (torch.randn(E, *s, chan, generator=g, dtype=torch.float64) for s in ((), (3,), (3, 3)))
+    along1, along2 = torch.einsum("ex,exc->ec", rh.double(), l1), torch.einsum("ey,exyc->exc", rh.double(), l2)
+    on_edge1, on_edge2 = along1[:, None] * rh.double()[:, :, None], along2[:, :, None] * rh.double()[:, None, :, None]
+    if features != "any":
+        l1, l2 = (on_edge1, on_edge2) if features == "along" else (l1 - on_edge1, l2 - on_edge2)
+    l0, l1, l2 = l0.float(), l1.float(), l2.float()
+    enc, encW, encb = torch.randn(E, 8, generator=g), torch.randn(chan, 8, generator=g) * 0.3, torch.randn(chan, generator=g)
+    row_ptr = (torch.arange(E + 1) * neighbours).clamp(max=E).int()
+
+    fma = lambda a, b, c: (a.double() * b.double() + c.double()).float()
+    phi = encb.expand(E, chan)
+    for m in range(8):
+        phi = fma(encW[:, m], enc[:, m:m + 1], phi)
+
+    def products(f, phi, l0, l1, l2, rh):
+        """The scalar products, and (coefficient, factor) of what is summed, in the arithmetic of f(a, b, c) = a b + c."""
+        dot = lambda v: f(v[2], rh[2], f(v[1], rh[1], v[0] * rh[0]))
+        cross = lambda v: [f(v[(x + 1) % 3], rh[(x + 2) % 3], -(v[(x + 2) % 3] * rh[(x + 1) % 3])) for x in range(3)]
+        t = [dot(l2[x]) for x in range(3)]
+        p = [phi * l0, phi * dot(l1), phi * dot(t)]
+        vectors = dict(zip(("011", "101", "121", "211", "111"),
+                           ([(p[0], rh[x]) for x in range(3)], [(phi, l1[x]) for x in range(3)], [(p[1], rh[x]) for x in range(3)],
+                            [(phi, t[x]) for x in range(3)], [(phi, c) for c in cross(l1)])))
+        pairs = [(x, y) for x in range(3) for y in range(3)]
+        rank2 = dict(zip(("022", "202", "112", "222", "212"),
+                         ([(p[0], rh[x] * rh[y]) for x, y in pairs], [(phi, l2[x][y]) for x, y in pairs], [(phi * l1[x], rh[y]) for x, y in pairs],
+                          [(phi * t[x], rh[y]) for x, y in pairs], [(phi, c) for x in range(3) for c in cross(l2[x])])))
+        return p, {**vectors, **rank2}
+
+    def by_component(dtype):
+        cast = lambda t: t.to(dtype)
+        return (cast(phi), cast(l0), [cast(l1[:, x]) for x in range(3)], [[cast(l2[:, x, y]) for y in range(3)] for x in range(3)],
+                [cast(rh[:, x:x + 1]) for x in range(3)])
+
+    p64, terms64 = products(lambda a, b, c: a * b + c, *by_component(torch.float64))
+    p32, terms32 = products(fma, *by_component(torch.float32))
+    per_node = lambda t: t.expand(E, chan).reshape(N, neighbours, chan)
+    sums = {}
+    for label, terms in terms32.items():
+        exact = torch.stack([per_node(a * b).sum(1) for a, b in terms64[label]], 1)
+        one_by_one = []
+        for a, b in terms:
+            a, b, s = per_node(a), per_node(b), torch.zeros(N, chan)
+            for k in range(neighbours):
+                s = fma(a[:, k], b[:, k], s)
+            one_by_one.append(s)
+        sums[label] = exact, torch.stack(one_by_one, 1)
+
+    def off(t):
+        flat = torch.cat([t.reshape(-1).float(), torch.zeros(1)]).cuda()   # (4 bytes past an aligned address: the path through registers)
+        return flat.roll(1)[1:].view(t.shape)
+
+    for place in (lambda t: t.contiguous().cuda(), off):
+        P0, S1, S2 = (t.cpu() for t in ops.bee_message(row_ptr.cuda(), torch.arange(E).int().cuda(), rh.cuda(), enc.cuda(), place(l0),
+                                                        place(l1), place(l2.reshape(E, 9, chan)), encW.cuda(), encb.cuda()))
+        results = [(lab, P0[:, k], p64[k], p32[k]) for k, lab in enumerate(("000", "110", "220"))]
+        for S, labels in ((S1, ("011", "101", "121", "211", "111")), (S2, ("022", "202", "112", "222", "212"))):
+            results += [(lab, S[:N, :, k], *sums[lab]) for k, lab in enumerate(labels)]
+        for label, got, exact, ours in results:
+            err, ref = (float((t.double() - exact).square().mean().sqrt()) for t in (got, ours))
+            print(f"[as exact] {features} {neighbours} {label}: {err:.3g}, one by one {ref:.3g}")
+            assert err <= 1.1 * ref, (label, err, ref)
+
+
 def test_node_products_emit_node_maxima(ops):
     g = torch.Generator().manual_seed(3)
     N, chan = 50, 128
