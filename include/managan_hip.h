@@ -975,7 +975,8 @@ int mg_group_norm(int mode, const float* x, long x_stride, const float* mul, lon
                   const float* res, void* scratch, float* out, mg_stream_t stream);
 /* Gradients of mode 0 for dense x and dy (batch, nodes, chan, comps), nothing added: dx like x, dgamma (chan).  scratch: what the
  * forward call of this x left there. */
-int mg_tensor_norm_grad_workspace_bytes(int batch, int chan, int groups, int comps, size_t* bytes /* host */);
+int mg_tensor_norm_grad_workspace_bytes(int batch, int chan, int groups, int comps, size_t* bytes /* host */);   /* any nodes */
+int mg_tensor_norm_grad_workspace_bytes_of(int batch, int nodes, int chan, int groups, int comps, size_t* bytes /* host */);
 int mg_tensor_norm_grad(const float* dy, const float* x, int batch, int nodes, int chan, int groups, int comps, float eps,
                         const float* gamma, const void* scratch, void* workspace, float* dx, float* dgamma, mg_stream_t stream);
 /* tens_sigmoid (managan/tensor_products.py:167-182): x / sqrt(1 + sum_comp x^2) per (row, chan). */

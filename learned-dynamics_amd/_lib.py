@@ -109,6 +109,7 @@ _SIGNATURES = {
     "mg_get_linear_mode": [],
     "mg_group_norm_scratch_bytes": [i32, i32, ctypes.POINTER(ctypes.c_size_t)],
     "mg_tensor_norm_grad_workspace_bytes": [i32, i32, i32, i32, ctypes.POINTER(ctypes.c_size_t)],
+    "mg_tensor_norm_grad_workspace_bytes_of": [i32, i32, i32, i32, i32, ctypes.POINTER(ctypes.c_size_t)],
     "mg_tensor_norm_grad": [vp, vp, i32, i32, i32, i32, i32, f32, vp, vp, vp, vp, vp, vp],
     "mg_group_norm": [i32, vp, i64, vp, i64, i32, i32, i32, i32, i32, f32, vp, vp, vp, i64, vp, vp, vp, vp],
     "mg_tens_sigmoid": [i32, vp, i64, vp, vp],

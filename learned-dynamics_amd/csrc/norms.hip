@@ -188,12 +188,15 @@ __global__ void __launch_bounds__(256) group_apply_kernel(const float* __restric
 //     dgamma[c] = sum dy x / s,   dx = gamma dy / s - x D / (s^3 count),   D = sum over the group of gamma dy x.
 // One pass sums dy x per channel position over chunks of a box's nodes, a second folds them group by group, a third forms dx:
 // 8192 nodes of 256 channels 21 us where a dozen of torch's passes took 130.  Both sums in fp64.
+// Chunks of a box: of four nodes, the loads that a thread has on its way at once, or as many as make 64 of them.  (64 for boxes of any
+// size asked for 545 MB beside 84 MB of x for 4096 boxes of 20 nodes and 256 channels; so 42.)
+int grad_chunks(int N) { return N < 4 * kChunks ? (int)ceil_div(N, 4) : kChunks; }
 // sums: [b][k][chunk]
 __global__ void __launch_bounds__(256) tensor_norm_grad_sums_kernel(const float* __restrict__ dy, const float* __restrict__ x, int N,
                                                                     int CT, double* __restrict__ sums) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.z, chunk = blockIdx.y;
+    const int k = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.z, chunk = blockIdx.y, chunks = gridDim.y;
     if (k >= CT) return;
-    const int per = (N + kChunks - 1) / kChunks, lo = chunk * per, hi = lo + per < N ? lo + per : N;
+    const int per = (N + chunks - 1) / chunks, lo = chunk * per, hi = lo + per < N ? lo + per : N;
     const long at = (long)b * N * CT + k;
     double sum = 0.0;
     int i = lo;
@@ -208,11 +211,11 @@ __global__ void __launch_bounds__(256) tensor_norm_grad_sums_kernel(const float*
         for (int u = 0; u < 4; u++) sum += (double)g[u] * v[u];
     }
     for (; i < hi; i++) sum += (double)dy[at + (long)i * CT] * x[at + (long)i * CT];
-    sums[((long)b * CT + k) * kChunks + chunk] = sum;
+    sums[((long)b * CT + k) * chunks + chunk] = sum;
 }
 
 // A workgroup to a (group, box).  coef[b groups + g] = (1 / s, D / (s^3 count)); of_box[b chan + c] = sum over the box of dy x / s
-__global__ void __launch_bounds__(256) tensor_norm_grad_fold_kernel(const double* __restrict__ sums, const double* __restrict__ partial,
+__global__ void __launch_bounds__(256) tensor_norm_grad_fold_kernel(const double* __restrict__ sums, int chunks, const double* __restrict__ partial,
                                                                     const float* __restrict__ gamma, int N, int chan, int groups, int T,
                                                                     float eps, float2* __restrict__ coef, double* __restrict__ of_box) {
     __shared__ double of_wave[4];
@@ -222,7 +225,7 @@ __global__ void __launch_bounds__(256) tensor_norm_grad_fold_kernel(const double
     double d = 0.0;
     for (int c = g * cg + wave; c < (g + 1) * cg; c += 4) {
         double q = 0.0;
-        for (int t = 0; t < T; t++) q += sums[((long)b * chan * T + (long)c * T + t) * kChunks + lane];
+        for (int t = 0; t < T; t++) q += lane < chunks ? sums[((long)b * chan * T + (long)c * T + t) * chunks + lane] : 0.0;
 #pragma unroll
         for (int e = kWave / 2; e > 0; e >>= 1) q += __shfl_xor(q, e);
         d += (double)gamma[c] * q;
@@ -398,10 +401,14 @@ int mg_painn_update_post(const float* lrv, int lrv_comp_major, const float* ip, 
                       1 + lrv_comp_major, UpdateVec{lrv, y, res_v, out_v}, stream);
 }
 
-int mg_tensor_norm_grad_workspace_bytes(int batch, int chan, int groups, int comps, size_t* bytes) {
-    MG_REQUIRE(bytes && batch >= 0 && chan >= 0 && groups >= 0 && comps >= 0, "mg_tensor_norm_grad_workspace_bytes: bad argument");
-    *bytes = (size_t)batch * chan * (comps * kChunks + 1) * sizeof(double) + (size_t)batch * groups * sizeof(float2);
+int mg_tensor_norm_grad_workspace_bytes_of(int batch, int nodes, int chan, int groups, int comps, size_t* bytes) {
+    MG_REQUIRE(bytes && batch >= 0 && nodes >= 0 && chan >= 0 && groups >= 0 && comps >= 0, "mg_tensor_norm_grad_workspace_bytes: bad argument");
+    *bytes = (size_t)batch * chan * ((size_t)comps * grad_chunks(nodes) + 1) * sizeof(double) + (size_t)batch * groups * sizeof(float2);
     return MG_OK;
+}
+
+int mg_tensor_norm_grad_workspace_bytes(int batch, int chan, int groups, int comps, size_t* bytes) {
+    return mg_tensor_norm_grad_workspace_bytes_of(batch, 4 * kChunks, chan, groups, comps, bytes);
 }
 
 int mg_tensor_norm_grad(const float* dy, const float* x, int batch, int nodes, int chan, int groups, int comps, float eps,
@@ -412,13 +419,13 @@ int mg_tensor_norm_grad(const float* dy, const float* x, int batch, int nodes, i
     MG_REQUIRE(dy && x && gamma && scratch && workspace && dx && dgamma, "mg_tensor_norm_grad: null pointer");
     MG_REQUIRE(batch <= 65535 && (long)chan * comps <= 0x7fffffffL, "mg_tensor_norm_grad: more than 65535 boxes");
     hipStream_t st = (hipStream_t)stream;
-    const int CT = chan * comps;
-    double *sums = static_cast<double*>(workspace), *of_box = sums + (long)batch * CT * kChunks;
+    const int CT = chan * comps, chunks = grad_chunks(nodes);
+    double *sums = static_cast<double*>(workspace), *of_box = sums + (long)batch * CT * chunks;
     float2* coef = reinterpret_cast<float2*>(of_box + (long)batch * chan);
     int threads;
     const dim3 grid = apply_grid(batch, nodes, CT, &threads);
-    hipLaunchKernelGGL(tensor_norm_grad_sums_kernel, dim3(grid.x, kChunks, grid.z), dim3(threads), 0, st, dy, x, nodes, CT, sums);
-    hipLaunchKernelGGL(tensor_norm_grad_fold_kernel, dim3((unsigned)groups, (unsigned)batch), dim3(256), 0, st, sums,
+    hipLaunchKernelGGL(tensor_norm_grad_sums_kernel, dim3(grid.x, (unsigned)chunks, grid.z), dim3(threads), 0, st, dy, x, nodes, CT, sums);
+    hipLaunchKernelGGL(tensor_norm_grad_fold_kernel, dim3((unsigned)groups, (unsigned)batch), dim3(256), 0, st, sums, chunks,
                        static_cast<const double*>(scratch), gamma, nodes, chan, groups, comps, eps, coef, of_box);
     hipLaunchKernelGGL(tensor_norm_grad_apply_kernel, grid, dim3(threads), 0, st, dy, x, batch, nodes, chan, groups, comps, gamma, coef, of_box,
                        dx, dgamma);

@@ -683,7 +683,7 @@ std::tuple<at::Tensor, at::Tensor> tens_norm_bwd(const at::Tensor& dy, const at:
     const int64_t B = x.size(0), N = x.size(1), C = x.size(2), T = x.numel() / (B * N * C);
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     size_t n = 0, kept = 0;
-    check(mg_tensor_norm_grad_workspace_bytes((int)B, (int)C, groups, (int)T, &n));
+    check(mg_tensor_norm_grad_workspace_bytes_of((int)B, (int)N, (int)C, groups, (int)T, &n));
     check(mg_group_norm_scratch_bytes((int)B, groups, &kept));
     TORCH_CHECK(scratch.is_cuda() && scratch.is_contiguous() && (size_t)scratch.nbytes() >= kept, "tens_norm_bwd: the sums of the forward pass");
     at::Tensor ws = bytes_like(x, n), dx = floats(x, x.sizes()), dgamma = floats(x, gamma.sizes());

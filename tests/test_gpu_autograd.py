@@ -1610,3 +1610,32 @@ def test_message_with_tangents_on_the_weights_of_its_node_mlp(pkg, residual):
         assert t is not None and t_ref is not None and float(t_ref.detach().norm()) > 0
         for a, b in ((p, p_ref), (t, t_ref)):
             assert float((a - b).detach().norm()) <= 1e-5 * float(b.detach().norm())
+
+
+@pytest.mark.parametrize("batch, nodes, chan, inds", [(3, 1, 16, 1), (2, 4, 16, 2), (70, 20, 64, 0), (2, 253, 16, 1), (2, 257, 16, 1),
+                                                      (1, 1030, 32, 0)])
+def test_tensor_norm_gradient_in_a_workspace_of_the_boxes_size(ops, batch, nodes, chan, inds):
+    """Chunks of a box by its nodes: gradients against float64, nothing written behind the workspace, which for small boxes is smaller
+    than what x takes."""
+    import ctypes
+    L = importlib.import_module("learned-dynamics_amd._lib")
+    diff = importlib.import_module("learned-dynamics_amd.differentiable")
+    lib, groups, comps = L.load(), 4, 3 ** inds
+    g = torch.Generator().manual_seed(nodes)
+    x, dy = (torch.randn(batch, nodes, chan, *[3] * inds, generator=g).cuda() for _ in range(2))
+    gamma = torch.randn(chan, *[1] * inds, generator=g).cuda()
+    y, kept = ops.tens_norm_fwd(x, gamma, groups, 1e-5)
+    size, any_nodes = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    L.check(lib.mg_tensor_norm_grad_workspace_bytes_of(batch, nodes, chan, groups, comps, ctypes.byref(size)))
+    L.check(lib.mg_tensor_norm_grad_workspace_bytes(batch, chan, groups, comps, ctypes.byref(any_nodes)))
+    assert size.value <= any_nodes.value and (nodes >= 253 or size.value <= 8 * batch * (chan * comps * (nodes + 7) // 4 + chan + groups))
+    workspace = torch.full((size.value // 4 + 4096,), -7, dtype=torch.int32, device="cuda")
+    dx, dgamma = torch.empty_like(x), torch.empty_like(gamma)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    L.check(lib.mg_tensor_norm_grad(p(dy), p(x), batch, nodes, chan, groups, comps, 1e-5, p(gamma), p(kept), p(workspace), p(dx), p(dgamma),
+                                    ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert bool((workspace[size.value // 4:] == -7).all())
+    leaves = [t.double().cpu().requires_grad_() for t in (x, gamma)]
+    want = torch.autograd.grad(diff._tens_norm_plain(*leaves, groups, 1e-5), leaves, dy.double().cpu())
+    for a, b in zip((dx, dgamma), want):                                 # (a handful of roundings to fp32 of sums in fp64)
+        assert float((a.double().cpu() - b).norm()) <= 4 * 2.0 ** -24 * float(b.norm())
