@@ -444,7 +444,10 @@ class _TensNorm(torch.autograd.Function):
         need = ctx.needs_input_grad[:2]
         if dy is None:
             return None, None, None, None
-        pieces = _gradients_in_pieces(lambda x, g: (_tens_norm_plain(x, g, ctx.groups, ctx.eps),), (x, gamma), need, (dy,))
+        f = lambda x, g: (_tens_norm_plain(x, g, ctx.groups, ctx.eps),)
+        if not torch._C._has_storage(dy):                                   # (a batch of gradients under vmap: is_grads_batched)
+            return _recorded_gradients(f, (x, gamma), need, (dy,)) + (None, None)
+        pieces = _gradients_in_pieces(f, (x, gamma), need, (dy,))
         if pieces is not None:
             return pieces + (None, None)
         dx, dgamma = ops.tens_norm_bwd(dy.contiguous(), x, gamma, sums, ctx.groups, ctx.eps)

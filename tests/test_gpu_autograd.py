@@ -1639,3 +1639,17 @@ def test_tensor_norm_gradient_in_a_workspace_of_the_boxes_size(ops, batch, nodes
     want = torch.autograd.grad(diff._tens_norm_plain(*leaves, groups, 1e-5), leaves, dy.double().cpu())
     for a, b in zip((dx, dgamma), want):                                 # (a handful of roundings to fp32 of sums in fp64)
         assert float((a.double().cpu() - b).norm()) <= 4 * 2.0 ** -24 * float(b.norm())
+
+
+def test_tensor_norm_with_a_batch_of_gradients(pkg):
+    """torch.autograd.grad(.., is_grads_batched=True), whose gradients have no memory that a kernel could read, against one at a time."""
+    tp = importlib.import_module("learned-dynamics_amd.tensor_products")
+    g = torch.Generator().manual_seed(7)
+    norm = tp.TensGroupNorm(1, 16, 4).cuda()
+    x = torch.randn(2, 50, 16, 3, generator=g).cuda().requires_grad_()
+    dys = torch.randn(3, 2, 50, 16, 3, generator=g).cuda()
+    y = norm(x)
+    together = torch.autograd.grad(y, (x, norm.gamma), dys, is_grads_batched=True, retain_graph=True)
+    for k, dy in enumerate(dys):
+        for a, b in zip(together, torch.autograd.grad(y, (x, norm.gamma), dy, retain_graph=True)):
+            assert float((a[k] - b).norm()) <= 1e-6 * float(b.norm())
