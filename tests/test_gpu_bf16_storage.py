@@ -74,8 +74,33 @@ def test_linear_bf16_onto_bf16_rows(ops, rows, dim_in, dim_out, act):
     _close_bf16(y, old.double() + (torch.where(pre > 0, pre, 0.1 * pre) if act == 2 else pre))
 
 
+@pytest.mark.parametrize("N, dims", [(600, (128, 128, 128, 128)), (130, (64, 96, 32, 64)), (1, (32, 32, 32, 64))])
+def test_messages_bf16_onto_their_features(pkg, N, dims):
+    """messages_forward(onto=True) against the increments of onto=False added outside: rounded once, s + B, where the increment was
+    rounded before the sum was: half an ulp of either apart, 2^-8 of a number at the lower end of its binade.  The vectors and
+    matrices in place, the scalars not."""
+    b16, bl, gl = (importlib.import_module(f"learned-dynamics_amd.{m}") for m in ("bee_layers_bf16", "bee_layers", "graph_layers"))
+    g = torch.Generator().manual_seed(N)
+    torch.manual_seed(N)
+    mod, E = bl.Messages(5.0, *dims).cuda(), 20 * N
+    src = torch.sort(torch.randint(0, N, (E,), generator=g)).values
+    graph = gl.Graph(src.cuda(), torch.randint(0, N, (E,), generator=g).cuda(), None, 1, N)
+    r = (torch.randn(E, 3, generator=g) * 1.5).cuda()
+    s = b16.to_storage(*(torch.randn(1, N, d, *[3] * k, generator=g).cuda() for k, d in enumerate(dims[:3])))
+    kept = [t.clone() for t in s]
+    with torch.no_grad():
+        apart = b16.messages_forward(mod, graph, r, *s)
+        assert all(torch.equal(a, b) for a, b in zip(s, kept))
+        onto = b16.messages_forward(mod, graph, r, *s, onto=True)
+    assert torch.equal(s[0], kept[0]) and torch.equal(onto[0], kept[0] + apart[0])
+    for y, mine, old, d in zip(onto[1:], s[1:], kept[1:], apart[1:]):
+        assert y.data_ptr() == mine.data_ptr() and float(d.float().abs().max()) > 0.01
+        old, d = old.double(), d.double()
+        assert bool(((y.double() - (old + d)).abs() <= 1.01 * 2.0 ** -8 * (d.abs() + (old + d).abs()) + 1e-6).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-def test_stack_bf16_keeps_its_inputs(pkg, dtype):
+def test_stack_bf16_keeps_its_inputs(pkg, dtype, monkeypatch):
     """The messages add to the features in place: to tensors of the stack's own, also where the inputs are bfloat16 and lie as the
     storage does (one channel)."""
     b16, bl = (importlib.import_module(f"learned-dynamics_amd.{m}") for m in ("bee_layers_bf16", "bee_layers"))
@@ -86,12 +111,9 @@ def test_stack_bf16_keeps_its_inputs(pkg, dtype):
         assert onto
         seen.append([t.clone() for t in (s_a, s_v, s_d)])
         return s_a + 1, s_v.add_(1), s_d.add_(1)
-    real = b16.messages_forward, b16.self_tens_prods_forward
-    b16.messages_forward, b16.self_tens_prods_forward = messages, lambda mod, a, v, d, batch, residual: (a, v, d)
-    try:
-        out = b16.stack_forward([None, None], [None, None], None, None, x_a, x_v, x_d)
-    finally:
-        b16.messages_forward, b16.self_tens_prods_forward = real
+    monkeypatch.setattr(b16, "messages_forward", messages)
+    monkeypatch.setattr(b16, "self_tens_prods_forward", lambda mod, a, v, d, batch, residual: (a, v, d))
+    out = b16.stack_forward([None, None], [None, None], None, None, x_a, x_v, x_d)
     assert all(torch.equal(a, b) for a, b in zip((x_a, x_v, x_d), kept))
     assert len(seen) == 2 and all(o.shape == k.shape and o.dtype == torch.float32 for o, k in zip(out, kept))
 

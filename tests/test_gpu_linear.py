@@ -626,8 +626,10 @@ def test_weight_gradient_with_one_narrow_dimension(ops, inds, rows, dims):
                                                  (40, 96, 40), (60000, 64, 128)])
 def test_linear_that_finds_its_own_row_maxima(ops, rows, dim_in, dim_out):
     """Without bounds the results are those with the exact row maxima to the bit, on either side of the line to reductions split over
-    waves, fewer pieces of a row than waves and more; a layer behind it scales by the maxima that it wrote.  Rows of zeros, of small
-    numbers, with infinities and NaN."""
+    waves, fewer pieces of a row than waves and more; the maxima are those of a pass of its own, and a layer behind it scales by them.
+    Rows of zeros, of small numbers, with infinities and NaN."""
+    L = importlib.import_module("learned-dynamics_amd._lib")
+    lib = L.load()
     g = torch.Generator().manual_seed(rows + dim_in)
     W, b = (torch.randn(dim_out, dim_in, generator=g) * dim_in ** -0.5).cuda(), torch.randn(dim_out, generator=g).cuda()
     W2, b2 = (torch.randn(dim_out, dim_out, generator=g) * dim_out ** -0.5).cuda(), torch.randn(dim_out, generator=g).cuda()
@@ -637,9 +639,28 @@ def test_linear_that_finds_its_own_row_maxima(ops, rows, dim_in, dim_out):
     x = x.cuda()
     bound = ops.row_absmax(x)
     same = lambda a, b: torch.equal(a.nan_to_num(1.5), b.nan_to_num(1.5))
+    planes, (y, maxima) = ops.packed_weight_f16x2(W), (torch.full((rows, n), -1.0, device="cuda") for n in (dim_out, 1))
+    args = _F16x2Linear(packed_W=planes.data_ptr(), x=x.data_ptr(), rows=rows, dim_in=dim_in, dim_out=dim_out, bias=b.data_ptr(), bias_rows=rows,
+                        out_comps=1, y=y.data_ptr())
+    L.check(lib.mg_tensor_linear_f16x2_run_unbounded(ctypes.byref(args), ctypes.c_void_p(maxima.data_ptr()),
+                                                     ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert torch.equal(maxima, bound)
+    given = y.clone()
+    args.x_rowmax, args.x_rowmax_parts, args.x_rowmax_stride, args.x_rows_per_bound, args.bound_mul = bound.data_ptr(), 1, 1, 1, 1.0
+    args.y = given.data_ptr()
+    L.check(lib.mg_tensor_linear_f16x2_run(ctypes.byref(args), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert same(y, given) and torch.isfinite(y).any()
     assert same(ops.tensor_linear_fwd(0, W, x, bias=b), ops.tensor_linear_fwd(0, W, x, bias=b, row_bound=bound))
     acts = [ops.ACT_SILU, ops.ACT_NONE]
     assert same(ops._ext.linear_chain(x, [W, W2], [b, b2], acts, None, 1.0, 0.0), ops._ext.linear_chain(x, [W, W2], [b, b2], acts, bound, 1.0, 0.0))
+
+
+class _F16x2Linear(ctypes.Structure):
+    _fields_ = [("packed_W", ctypes.c_void_p), ("x", ctypes.c_void_p), ("x_rowmax", ctypes.c_void_p), ("x_rowmax_parts", ctypes.c_int),
+                ("x_rowmax_stride", ctypes.c_long), ("x_rows_per_bound", ctypes.c_long), ("bound_mul", ctypes.c_float),
+                ("bound_add", ctypes.c_float), ("rows", ctypes.c_long), ("dim_in", ctypes.c_int), ("dim_out", ctypes.c_int),
+                ("bias", ctypes.c_void_p), ("bias_rows", ctypes.c_long), ("act", ctypes.c_int), ("accumulate", ctypes.c_int),
+                ("out_comps", ctypes.c_int), ("sequential", ctypes.c_int), ("y", ctypes.c_void_p), ("y_rowmax", ctypes.c_void_p)]
 
 
 class _WgradJob(ctypes.Structure):
