@@ -408,8 +408,10 @@ std::tuple<at::Tensor, OptTensor> linear_fwd(int64_t inds, const at::Tensor& W, 
             TORCH_CHECK(row_bound->dim() == 2 && (row_bound->size(0) * rows_per == R || row_bound->size(0) == 1),
                         "row_bound must be (rows / rows_per_bound, parts)");
         } else {
-            // (a pass of its own: the binding's fp32 linear is to stay the cheaper call for small plain rows, 5.7 us of host time at
-            // 256 x 64 -> 64 in a process of many streams where this operator takes 5.2 without the pass; chains find theirs on the way)
+            // A pass of its own.  On the way it would be one launch less (256 x 64 -> 64: 3.9 us of the GPU and 5.9 of the host, 6.3 and
+            // 8.7 with the pass).  But the binding's fp32 linear, which promises less host time than this operator, is a kernel of
+            // 10.4 us there: 4.4 us a call while launches may queue up, 5.6 in processes where they wait for the GPU before that,
+            // where this operator then takes 5.3.  Chains and the linears of rows inside the layers find theirs on the way.
             b = Bound{row_absmax(x.reshape({R, dim_in}))};
         }
         run_f16x2(W, dim_in, fp(x), R, b, bias, act, accumulate, out_comps, y, rowmax_buffer(dim_in), sequential);
