@@ -278,8 +278,11 @@ constexpr int kFBuf = 4 * kFPlane;                 // one stage: two operands x 
 constexpr int kFParts = 1024;                      // partial maxima per operand
 // rows per accumulation run (a multiple of kFRows).  Slices get longer the more tiles a product has: 27 000 rows of 16 x 1280 are
 // 1080 a slice, whose weights' gradients were off by 4.8e-7 of their 2-norm in one run and are by 3.4e-7 in runs of 256 (as the
-// five products of 16 x 256, 211 rows a slice, were); the additions do not show in the time.
-constexpr int kFRun = 256;
+// five products of 16 x 256, 211 rows a slice, were).  Runs of 128 took 4096 x 512 x 512 from 2.0e-7 to 1.6e-7 and 5000 rows of 64 x 256
+// beside two of 256 x 256 from 2.5e-7 to 2.3e-7, for half a percent of a training step at most.  The column sums go by the same runs: in one
+// chain a slice, 78 000 rows of an MLP's three layers were off by 4.6e-7 of the 2-norm product by product, by 6.4e-7 together, whose slices are
+// longer, and are by 1.8e-7.
+constexpr int kFRun = 128;
 
 // parts[b] = max |x| over the b-th share of n floats (n % 4 == 0, x 16-byte aligned)
 __global__ void __launch_bounds__(256) absmax_parts_kernel(const float* __restrict__ x, long n,
@@ -406,7 +409,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     };
     // column sums of dy over the slice (the bias gradient), by the workgroups of the first column of tiles
     const bool sum_cols = job.colsum >= 0 && i_tile == 0;                          // (uniform)
-    float4 colsum = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 colsum = make_float4(0.f, 0.f, 0.f, 0.f), colsums = colsum;             // (of a run of stages, of the runs before it)
     // One stage in eight parts: part g splits columns 2 (g % 2) and one more of rows 2 (g / 2) and one more of the stage at r, which
     // are in v or on their way there; every second part requests the same two rows of the stage at r_next.  finish writes the pieces.
     struct Pieces {
@@ -573,6 +576,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
                 for (int q = 0; q < 2; q++)
 #pragma unroll
                     for (int k = 0; k < 16; k++) { total[p][q][k] += acc[p][q][k]; acc[p][q][k] = 0.f; }
+            if constexpr (decltype(sums)::value) {
+                colsums.x += colsum.x; colsums.y += colsum.y; colsums.z += colsum.z; colsums.w += colsum.w;
+                colsum = make_float4(0.f, 0.f, 0.f, 0.f);
+            }
         }
     };
     fetch(r_lo);
@@ -583,7 +590,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     if (sum_cols) {
         // the four row groups of a column quad, added in a fixed order
         float4* sums = reinterpret_cast<float4*>(lds);                             // [octet][cq]; the stage buffers are done with
-        if (!stage_x) sums[octet * 32 + cq] = colsum;
+        if (!stage_x) sums[octet * 32 + cq] = colsums;                             // (the stage behind the last run added nothing)
         __syncthreads();
         if (threadIdx.x < 32) {
             const float4 s0 = sums[cq], s1 = sums[32 + cq], s2 = sums[64 + cq], s3 = sums[96 + cq];
@@ -666,16 +673,15 @@ __global__ void __launch_bounds__(256) wgrad_reduce_f16x2_kernel(const float4* _
     if constexpr (MANY) s = sum_of_slices(part, quads, splits, k, shared);
     if (k >= quads || (MANY && threadIdx.x >= 16)) return;
     if constexpr (!MANY) {
-    auto add = [&](const float4& v) { s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w; };
-    int z = 0;
-    for (; z + 8 <= splits; z += 8) {                      // eight loads in flight, added in slice order
-        float4 v[8];
+        auto plus = [](const float4& a, const float4& b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); };
+        int z = 0;
+        for (; z + 8 <= splits; z += 8) {                  // eight loads in flight, added in pairs
+            float4 v[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) v[u] = part[(long)(z + u) * quads + k];
-#pragma unroll
-        for (int u = 0; u < 8; u++) add(v[u]);
-    }
-    for (; z < splits; z++) add(part[(long)z * quads + k]);
+            for (int u = 0; u < 8; u++) v[u] = part[(long)(z + u) * quads + k];
+            s = plus(s, plus(plus(plus(v[0], v[1]), plus(v[2], v[3])), plus(plus(v[4], v[5]), plus(v[6], v[7]))));
+        }
+        for (; z < splits; z++) s = plus(s, part[(long)z * quads + k]);
     }
     float* out = seg.out[0];
     int first = 0;
@@ -969,8 +975,9 @@ int mg_tensor_linear_wgrad_f16x2_supported(long rows, int dim_in, int dim_out) {
 // slices.  What a launch costs beside its products, the bounds that every workgroup reads, the first loads, the partial results of
 // as many workgroups as the chip holds and their sum, is then paid once, and the slices are longer: the three products of
 // an MLP 128 -> 512 -> 512 -> 512 at 4096 rows 77 -> 39 us, at 8192 92 -> 56, at 32 768 242 -> 183, at 155 744 806 -> 758; four of
-// 256 x 256 at 24 576 141 -> 76; 512 x 1024 and two of 1024 x 1024 at 8192 (two launches) 204 -> 194.  Errors against float64 are those of
-// single products or less.
+// 256 x 256 at 24 576 141 -> 76; 512 x 1024 and two of 1024 x 1024 at 8192 (two launches) 204 -> 194.  The longer slices cost
+// up to 15 % in the error of a narrow product (128 -> 512 at 4096 rows 1.6e-7 of its 2-norm from float64, singly 1.4e-7) and 25 % in the column
+// sums (1.7e-7, 1.4e-7 at 78 000 rows), in runs of kFRun rows both.
 constexpr long kMergedTiles = 128;
 static long job_tiles(const mg_wgrad_f16x2& j) { return ceil_div(j.dim_out, kFTile) * ceil_div(j.dim_in, kFTile); }
 static int together(const mg_wgrad_f16x2* jobs, int count) {

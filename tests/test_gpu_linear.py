@@ -708,6 +708,34 @@ def test_weight_gradients_of_several_layers_in_one_launch(ops, rows, dims):
 
 
 
+@pytest.mark.parametrize("rows", [4096, 78000])
+def test_gradients_of_several_layers_in_one_launch_in_short_chains(ops, rows):
+    """The three layers of an MLP of 512 columns: together the slices of rows are longer, the chains in which they are summed are not.
+    Column sums: chains of 32 numbers, of as many runs as a slice has (44 at most here) and of 14 slices in eights, which for random
+    numbers are off by 2^-24 (32 / 6 + 44 / 6 + 3)^(1/2) = 4 x 2^-24 of their 2-norm: 5 x 2^-24.  Products: within a
+    fifth of the error that they have singly in shorter slices (a chain twice as long is off by a fifth more where half of the
+    error is the pieces')."""
+    L = importlib.import_module("learned-dynamics_amd._lib")
+    lib, g = L.load(), torch.Generator(device="cuda").manual_seed(rows)
+    dims, jobs, held = [(128, 512), (512, 512), (512, 512)], (_WgradJob * 3)(), []
+    for k, (dim_in, dim_out) in enumerate(dims):
+        x, dy = (torch.randn(rows, d, device="cuda", generator=g) for d in (dim_in, dim_out))
+        dW, db = torch.empty(dim_out, dim_in, device="cuda"), torch.empty(dim_out, device="cuda")
+        jobs[k] = _WgradJob(dy.data_ptr(), x.data_ptr(), None, 0, None, 0, rows, dim_in, dim_out, dW.data_ptr(), db.data_ptr())
+        held.append((x, dy, dW, db))
+    size = ctypes.c_size_t()
+    L.check(lib.mg_tensor_linear_wgrad_f16x2_many_workspace_bytes(ctypes.byref(jobs), 3, rows, ctypes.byref(size)))
+    ws = torch.empty(size.value, dtype=torch.uint8, device="cuda")
+    L.check(lib.mg_tensor_linear_wgrad_f16x2_many(ctypes.byref(jobs), 3, rows, ws.data_ptr(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    off = lambda t, ref: float((t.double() - ref).norm() / ref.norm())
+    for x, dy, dW, db in held:
+        one, one_b = ops.tensor_linear_wgrad(0, dy, x, want_bias=True)
+        ref, ref_b = dy.double().t() @ x.double(), dy.double().sum(0)
+        print(f"[together / singly] {rows}: dW {off(dW, ref):.3g} / {off(one, ref):.3g}, db {off(db, ref_b):.3g} / {off(one_b, ref_b):.3g}")
+        assert off(db, ref_b) <= 5 * 2.0 ** -24 and off(one_b, ref_b) <= 5 * 2.0 ** -24
+        assert off(dW, ref) <= 1.2 * off(one, ref)
+
+
 def test_weight_gradient_at_the_edge_count_of_configs2(ops):
     """The split-fp16 weight gradient at the size training runs it at (1592454 edge rows, 512 x 512): against float64
     accumulated over row chunks on the device, with the error of torch's own fp32 product of the same operands as
