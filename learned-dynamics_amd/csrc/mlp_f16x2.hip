@@ -558,12 +558,14 @@ int launch(const MlpArgs& a, hipStream_t st) {
     return check_launch("mg_mlp_f16x2");
 }
 
+// 32 rows a workgroup while the chip holds all of them at once, 64 beyond (the weights are read half as often):
+// 128 -> 512 on 8192 rows 42 against 53 us, on 16 336 83 against 69; 128 -> 128 on 16 336 14.5 against 18.0
+bool wide_tiles(const MlpArgs& a) { return ceil_div(a.R, 32) * (a.O / 32) > 256 * kMaxWaves; }
+
 template <int MODE>
 int choose(const MlpArgs& a, bool dual, hipStream_t st) {
     if constexpr (MODE == kInfer) {
-        // 32 rows a workgroup while the chip holds all of them at once, 64 beyond (the weights are read half as often):
-        // 128 -> 512 on 8192 rows 42 against 53 us, on 16 336 83 against 69; 128 -> 128 on 16 336 14.5 against 18.0
-        if (ceil_div(a.R, 32) * (a.O / 32) > 256 * kMaxWaves) return launch<2, 1, MODE, false>(a, st);
+        if (wide_tiles(a)) return launch<2, 1, MODE, false>(a, st);
         return launch<1, 1, MODE, false>(a, st);
     } else {
         // The passes over memory between the layers are longer here (z and h, or z and the gradients): from more tiles than CUs on two
@@ -656,20 +658,21 @@ int mg_mlp_f16x2_forward(const mg_mlp_f16x2* p, mg_stream_t stream) {
     return keep ? choose<kTrain>(a, p->dual, (hipStream_t)stream) : choose<kInfer>(a, false, (hipStream_t)stream);
 }
 
-// kMany to a launch
+// kMany to a launch, each MLP in the tiles that it has alone: 64 rows leave no registers for the small products' own sums, so that a
+// row would be less exact beside others (128 -> 512 2.25e-7 of the 2-norm from float64, 1.88e-7 in 32 rows)
 static int forward_many(const mg_mlp_f16x2* const* in, int jobs, hipStream_t st) {
-    if (jobs > kMany) {
-        if (int code = forward_many(in, kMany, st)) return code;
-        return forward_many(in + kMany, jobs - kMany, st);
-    }
-    MlpMany p{};
-    long tiles = 0;
-    int used = 0;
+    MlpMany p[2] = {};
+    int used[2] = {0, 0};
+    auto send = [&](int wide) {
+        const int count = used[wide];
+        used[wide] = 0;
+        return count == 0 ? MG_OK : wide ? launch_many<2>(p[1], count, st) : launch_many<1>(p[0], count, st);
+    };
     for (int k = 0; k < jobs; k++) {
         const mg_mlp_f16x2& m = *in[k];
         MG_REQUIRE(m.rows >= 0 && mg_mlp_f16x2_supported(m.dim_in, m.dim) && m.dim == in[0]->dim && !m.dual && !m.z[0] && !m.h[0] && !m.x_rowmax,
                    "mg_mlp_f16x2_forward_many: inference only, one width, dimensions multiples of 32 up to %d", kMaxDim);
-        MlpArgs& a = p.job[used];
+        MlpArgs a{};
         a.x = m.x;
         a.R = m.rows;
         a.K = m.dim_in;
@@ -681,13 +684,14 @@ static int forward_many(const mg_mlp_f16x2* const* in, int jobs, hipStream_t st)
         }
         MG_REQUIRE(fill(a, m.packed_W, a.K, a.O, a.N) && (m.rows == 0 || (a.x && a.y && aligned16(a.x) && aligned16(a.y))),
                    "mg_mlp_f16x2_forward_many: null or unaligned pointer");
-        tiles += ceil_div(m.rows, 32);
-        if (m.rows > 0) used++;
+        if (m.rows == 0) continue;
+        const int wide = wide_tiles(a);
+        p[wide].job[used[wide]++] = a;
+        if (used[wide] == kMany)
+            if (int code = send(wide)) return code;
     }
-    if (tiles == 0) return MG_OK;
-    // (the line of one MLP)
-    if (tiles * (in[0]->dim / 32) > 256 * kMaxWaves) return launch_many<2>(p, used, st);
-    return launch_many<1>(p, used, st);
+    if (int code = send(0)) return code;
+    return send(1);
 }
 
 int mg_mlp_f16x2_forward_many(const mg_mlp_f16x2* const* args, int count, mg_stream_t stream) {

@@ -474,3 +474,19 @@ def test_a_weight_beyond_the_pieces_in_one_of_two_mlps(ops, layer, value):
     one, other = ops.filter_grids((x, unit, W, b), (x, unit, bad, b))
     assert torch.equal(one, ops.filter_grid(x, unit, W, b))
     _assert_like(other, _formula(x.double(), bad, b), (layer, value))
+
+
+@pytest.mark.parametrize("n, rows", [(128, [6000] * 6), (128, [1100, 16000, 2000, 9000, 5000]), (64, [300, 20000, 5000, 7000]), (64, [700] * 33)])
+def test_filters_evaluated_together_are_those_evaluated_alone(pkg, ops, n, rows):
+    """More rows together than the chip holds in tiles of 32, some of them more by themselves, more MLPs than a launch takes: every one
+    the bits that it has alone."""
+    painn = importlib.import_module("learned-dynamics_amd.painn")
+    torch.manual_seed(n + len(rows))
+    jobs = []
+    with torch.no_grad():
+        for E in rows:
+            msg = painn.Message(5.0, n).cuda()
+            enc = ops.painn_radial_encode(torch.randn(E, 3, device="cuda") * 2, msg.n_rbf, 5.0)
+            jobs.append((enc, ops.linear_in_unit_bound(enc.device), *painn._plain_params(msg.mlp_dist)))
+        for y, job in zip(ops.filter_grids(*jobs), jobs):
+            assert torch.equal(y, ops.filter_grid(*job)), job[0].shape
