@@ -84,8 +84,8 @@ def _mlp_params(mlp):
 def _own_parameters(mlp):
     """The parameters that an MLP's filter depends on, to be stamped: out of the modules' dictionaries where the three linears are
     plain and hold theirs (a walk over the modules is 15 us), else whatever parameters() finds.  A weight that is computed at every
-    access (torch.nn.utils.parametrize) is a new tensor each time, often at the address of the one before: no stamp tells two
-    of them apart, those of the parameters that it is computed from do."""
+    access (torch.nn.utils.parametrize) is a new tensor each time, with another stamp; the stamps of the parameters that it is
+    computed from change when they do."""
     if type(mlp) is MLP:
         linears = list(mlp._modules["layers"]._modules.values())[0:5:2]
         if all(type(lin) is nn.Linear and {"weight", "bias"} <= lin._parameters.keys() for lin in linears):
