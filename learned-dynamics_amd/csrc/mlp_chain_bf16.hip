@@ -3,14 +3,20 @@
 //     psi = Y P0                      (edges, 128)      -> sum over the edges of each node of bf16(psi)
 //     h1  = act(W1 psi + b1)          (edges, 256)
 //     h2  = act(W2 h1 + b2)           (edges, 256)      -> sum over the edges of each node of bf16(h2)
-// in ONE kernel: psi, h1 and h2 never leave the registers.  With W as the first matrix operand an accumulator
-// register holds (edge = lane % 32, four consecutive channels), and that is also the layout the matrix core
-// wants for its second operand (16 of a 32-channel chunk's channels per lane half), up to a fixed permutation of
-// the channels inside a chunk which the caller applies to the input channels of W1 and W2 before packing.  So
-// the bf16-rounded outputs of one layer (rounded exactly where the separate kernels round them when they store)
-// are the operands of the next without any data movement.  Weights stream through LDS as in the plain kernel
-// (two bf16 planes, 16 significand bits); x = P0 is the only tensor read from HBM, the sums the only output.
-// Widths are fixed (128 -> 256 -> 256) by the register budget: 64 + 128 accumulators and 64 operand registers.
+// in ONE kernel: psi and h1 stay in LDS, h2 in registers; each is rounded to bf16 exactly where the separate kernels round it when
+// they store.  x = P0 is the only per-row tensor read, the sums the only output.  Weights are two bf16 planes (16 significand bits).
+//
+// A workgroup takes 128 rows through the three layers, two workgroups to a CU.  Activations lie in LDS in the order the matrix cores
+// read them (fragment_at); a wave owns 32 output columns and reads the fragments of its weights straight from memory: a step of 16 k
+// is two contiguous kilobytes of the L2 and feeds eight matrix instructions, and no barrier stands in the loop over k of the hidden
+// layers.  Where rows are the first operand (psi, h2) a lane of the product holds rows of one column, which a segment's sum adds up in
+// a register; where they are the second (h1) four consecutive channels of one row, the next layer's operand eight bytes at a time.
+//
+// 5.9 M rows of 384 with 90 to a segment 3.59 ms, 180 000 rows 0.125 ms; with psi, h1 and h2 in the registers of one wave per 32 rows
+// and the weights through LDS (two fragments read for two matrix instructions, a barrier for every 32 k) 4.11 and 0.134 ms.  What
+// bounds it: the board's power.  It takes 22 % fewer cycles than that kernel, the matrix cores are busy for half of them (0.97 PFLOP/s,
+// counting both planes), and the clock falls from 2.1 to 1.84 GHz.  64 columns to a wave and half the waves, a third less read for a
+// matrix instruction: 3.85 ms.  Writers of a row meeting in one bank (fragment_at without its turn): 3.66 ms.
 #include "common.hpp"
 #include "rowsum_finish.hpp"
 
@@ -19,16 +25,14 @@ namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kCK = 32;      // k per chunk (two MFMA steps)
-constexpr int kRowW = 80;    // bytes per LDS row of one W plane (64 + 16 pad)
-constexpr int kRB = 1;       // blocks of 32 rows per wave.  With 2 every W fragment read from LDS would feed two matrix
-                             // instructions, but 256 accumulators leave one wave per SIMD and nothing to hide the
-                             // loads and barriers behind: measured 4.7 ms against 2.0 ms at 2.26 M rows
-constexpr int kWaves = 8 / kRB, kThreads = 64 * kWaves;      // 256 rows per workgroup
 constexpr int kD = 128, kH = 256;
-constexpr int kLdsBytes = 2 * 2 * kH * kRowW;               // two buffers of two planes of 256 rows
-constexpr int kRed = 68;                                     // floats per row of a reduction slice
+constexpr int kBlocks = 4, kRows = 32 * kBlocks, kThreads = 512;  // row blocks and rows of a workgroup
+constexpr int kStage = 128, kStageBlock = 32 * kStage;            // k of x in LDS at a time; elements of a row block's part of it
+constexpr int kStageElems = kRows * kStage;                       // (psi has the place of a stage, h1 that of both)
+constexpr int kStep = 2 * 64 * 8;                                 // elements of a weight's fragments for 16 k: two planes
+constexpr int kPackedDimIn = 1024;                                // widest Y that the workspace has room for in fragments
 
 template <int ACT>
 __device__ __forceinline__ float activate_c(float v) {
@@ -37,292 +41,243 @@ __device__ __forceinline__ float activate_c(float v) {
     return v;
 }
 
-// Streams the two planes of W (rows n0 .. n0 + 32 NI of a (w_rows, I) packed matrix) through LDS chunk by chunk.
-template <int NI>
-struct WStream {
-    static constexpr int TN = 32 * NI, kPlaneW = TN * kRowW, kBufW = 2 * kPlaneW;
-    static constexpr int kPer = 8 * TN / kThreads;           // 16-byte pieces per thread and chunk
-    static_assert(TN % 128 == 0, "a thread's pieces must differ by whole planes and rows only");
-    const __bf16* src;                                        // piece j: + plane(j) plane_elems + row(j) I
-    long plane_elems;
-    int dst, I;
-    bf16x8 regs[kPer];
-    static constexpr int plane_of(int j) { return (kThreads * j) / (4 * TN); }
-    static constexpr int row_of(int j) { return ((kThreads * j) % (4 * TN)) / 4; }
-    __device__ __forceinline__ void init(const __bf16* Wp, long plane_elems_, int I_) {
-        I = I_;
-        plane_elems = plane_elems_;
-        const int tid = threadIdx.x;
-        src = Wp + (long)(tid >> 2) * I + 8 * (tid & 3);
-        dst = (tid >> 2) * kRowW + (tid & 3) * 16;
-    }
-    __device__ __forceinline__ void load(int k0) {
-        k0 = k0 < I ? k0 : I - kCK;                           // surplus requests past the end are never used
+// Element (row, k) of a row block: chunks of 32 k, in each two steps of 16, 8 consecutive k to a lane.  The four pieces of 8 k of a
+// chunk lie 512 bytes apart: the last two bits of the row are turned by the piece, so that writers of one row meet different banks.
+__device__ __forceinline__ int piece_of(int k) { return ((k >> 3) & 1) + 2 * ((k >> 4) & 1); }
+__device__ __forceinline__ int fragment_at(int row, int k) {
+    return (((k >> 5) * 2 + ((k >> 3) & 1)) * 64 + (row ^ piece_of(k)) + 32 * ((k >> 4) & 1)) * 8 + (k & 7);
+}
+
+// The two planes of a packed weight (rows of I; PERMUTED: the channels of a chunk in the order that mg_mlp_chain_bf16 asks for) into
+// fragments: [32 rows][16 k][plane][lane][8]
+struct Repack {
+    const __bf16* from;
+    long plane;
+    int rows, I, permuted;
+    __bf16* to;
+};
+struct RepackAll {
+    Repack w[3];
+};
+__global__ void __launch_bounds__(256) mlp_chain_repack_kernel(const RepackAll all) {
+    const Repack w = all.w[blockIdx.y];
+    const long t = (long)blockIdx.x * 256 + threadIdx.x;           // of rows I / 4: eight elements each
+    if (t >= (long)w.rows * w.I / 4) return;
+    const int lane = (int)(t & 63), plane = (int)(t >> 6) & 1, steps = w.I / 16;
+    const long step = t >> 7;
+    const int row = 32 * (int)(step / steps) + (lane & 31), s = (int)(step % steps);
+    const __bf16* from = w.from + plane * w.plane + (long)row * w.I + 32 * (s >> 1);
+    bf16x8 v;
 #pragma unroll
-        for (int j = 0; j < kPer; j++)
-            regs[j] = *reinterpret_cast<const bf16x8*>(src + plane_of(j) * plane_elems + (long)row_of(j) * I + k0);
+    for (int j = 0; j < 8; j++) {
+        const int ch = 16 * (lane >> 5) + 8 * (s & 1) + j;
+        v[j] = from[w.permuted ? 16 * ((ch >> 2) & 1) + 4 * (ch >> 3) + (ch & 3) : ch];
     }
-    __device__ __forceinline__ void store(unsigned char* buf) const {
-#pragma unroll
-        for (int j = 0; j < kPer; j++)
-            *reinterpret_cast<bf16x8*>(buf + dst + plane_of(j) * kPlaneW + row_of(j) * kRowW) = regs[j];
+    *reinterpret_cast<bf16x8*>(w.to + 8 * t) = v;
+}
+
+// acc[mi] += rows of block mi (from LDS) times 32 weight rows, a step of 16 k at a time; the weights of two steps are in flight.
+// ROWS_FIRST: a lane of acc is a column and its registers are rows 8 (q / 4) + 4 (lane / 32) + q % 4; else a row and its channels.
+// PLANES: the weight is read from its planes of rows, a line for every row: Y where the workspace has no room for its fragments.
+template <int MI, bool ROWS_FIRST, bool PLANES = false>
+struct Product {
+    floatx16 acc[MI];
+    const __bf16* w;
+    int steps, next;
+    unsigned lane_at;
+    long low;
+    bf16x8 wh[2], wl[2];
+    __device__ __forceinline__ void load_w(int u) {
+        const int s = next < steps ? next : steps - 1;             // (surplus loads at the end are never used)
+        const __bf16* p = w + (PLANES ? 32L * (s >> 1) + 8 * (s & 1) : (long)kStep * s);
+        wh[u] = *reinterpret_cast<const bf16x8*>(p + lane_at);
+        wl[u] = *reinterpret_cast<const bf16x8*>(p + low + lane_at);
+        next++;
     }
-    // acc[rb][ni] += W chunk (from buf) x the lane's 16 operand values of the chunk (two 8-value steps)
-    template <typename XOf>
-    __device__ __forceinline__ void multiply(floatx16 (&acc)[kRB][NI], const unsigned char* buf, XOf x_of) const {
+    // block: which 32 rows of the weight
+    __device__ __forceinline__ void start(const __bf16* weight, long plane, int block, int K) {
         const int lane = threadIdx.x & 63;
-        const int b_off = (lane & 31) * kRowW + 32 * (lane >> 5);
+        steps = K / 16;
+        next = 0;
+        w = weight + (long)block * (PLANES ? 32 * K : kStep * steps);
+        lane_at = PLANES ? (unsigned)((lane & 31) * K + 16 * (lane >> 5)) : 8u * lane;
+        low = PLANES ? plane : kStep / 2;
 #pragma unroll
-        for (int s = 0; s < 2; s++)
+        for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-            for (int ni = 0; ni < NI; ni++) {
-                const bf16x8 wh = *reinterpret_cast<const bf16x8*>(buf + b_off + ni * 32 * kRowW + 16 * s);
-                const bf16x8 wm = *reinterpret_cast<const bf16x8*>(buf + kPlaneW + b_off + ni * 32 * kRowW + 16 * s);
+            for (int q = 0; q < 16; q++) acc[mi][q] = 0.f;
+        load_w(0);
+        load_w(1);
+    }
+    __device__ __forceinline__ void run(const __bf16* x, int block_elems, int n) {      // n steps, an even number
+        const int lane = threadIdx.x & 63;
+        const __bf16* const at[2] = {x + fragment_at(lane & 31, 16 * (lane >> 5)), x + fragment_at(lane & 31, 16 * (lane >> 5) + 8)};   // of even and odd steps
+        bf16x8 b[MI];
 #pragma unroll
-                for (int rb = 0; rb < kRB; rb++) {
-                    acc[rb][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wm, x_of(rb, s), acc[rb][ni], 0, 0, 0);   // small term first
-                    acc[rb][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wh, x_of(rb, s), acc[rb][ni], 0, 0, 0);
+        for (int mi = 0; mi < MI; mi++) b[mi] = *reinterpret_cast<const bf16x8*>(at[0] + mi * block_elems);
+        for (int s = 0; s < n; s += 2) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int chunk = u && s + 2 < n ? s + 2 : s;          // (the last trip reads its own chunk again)
+#pragma unroll
+                for (int pair = 0; pair < MI; pair += 2) {
+                    __builtin_amdgcn_sched_barrier(0);             // keep this issue order
+#pragma unroll
+                    for (int mi = pair; mi < pair + 2; mi++) acc[mi] = product(wl[u], b[mi], acc[mi]);   // small terms first
+#pragma unroll
+                    for (int mi = pair; mi < pair + 2; mi++) acc[mi] = product(wh[u], b[mi], acc[mi]);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int mi = pair; mi < pair + 2; mi++)
+                        b[mi] = *reinterpret_cast<const bf16x8*>(at[1 - u] + mi * block_elems + 512 * chunk);
                 }
+                load_w(u);
             }
+        }
+    }
+    static __device__ __forceinline__ floatx16 product(const bf16x8& w, const bf16x8& x, const floatx16& c) {
+        return ROWS_FIRST ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, w, c, 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, x, c, 0, 0, 0);
     }
 };
 
-// act(acc + bias) of a layer with 32 NI channels, rounded to bf16: chunk c, step s -> the lane's eight operand
-// values for the next layer (accumulator registers 8 s .. 8 s + 7 of block c).  BIAS = false: no bias.
-template <int ACT, bool BIAS, int NI>
-__device__ __forceinline__ void to_operands(const floatx16 (&acc)[kRB][NI], const float* __restrict__ bias,
-                                            bf16x8 (&ops)[kRB][NI][2]) {
-    const int g = (threadIdx.x >> 5) & 1;
+// The sums over the rows of each segment, column `col`: v[half][q] are the lane's rows of two blocks as Product has them with
+// ROWS_FIRST.  Two partial slots per block of 32 rows (rowsum_finish.hpp); runs strictly inside a block are written to `out`.
+// After the halves have changed places lanes 0 .. 31 hold all rows of the first block and lanes 32 .. 63 those of the second, and a
+// segment's rows add up in row order.
+__device__ __forceinline__ void sum_segments(float (&v)[2][16], long first_block, long R, const int* __restrict__ seg, int O, int col,
+                                             float* __restrict__ slots, long n_blocks, float* __restrict__ out) {
+    const int lane = threadIdx.x & 63, m = lane & 31, G = lane >> 5;
 #pragma unroll
-    for (int c = 0; c < NI; c++) {
-        float4 b[4];
-#pragma unroll
-        for (int qq = 0; qq < 4; qq++)
-            b[qq] = BIAS ? *reinterpret_cast<const float4*>(bias + 32 * c + 8 * qq + 4 * g) : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (int rb = 0; rb < kRB; rb++)
-#pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const float v = activate_c<ACT>(acc[rb][c][q] + (&b[q / 4].x)[q % 4]);
-                ops[rb][c][q / 8][q % 8] = (__bf16)v;
-            }
-        __builtin_amdgcn_sched_barrier(0);                    // one block at a time: the registers are nearly all taken
+    for (int q = 0; q < 16; q++) {
+        const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[0][q]), __float_as_uint(v[1][q]), false, false);
+        v[0][q] = __uint_as_float(s[0]);                           // row 8 (q / 4) + q % 4 of block G
+        v[1][q] = __uint_as_float(s[1]);                           // row 8 (q / 4) + 4 + q % 4
     }
-}
-
-// layer whose operands are in registers: K = 32 NCH
-template <int NI, int NCH>
-__device__ __forceinline__ void layer_from_registers(floatx16 (&acc)[kRB][NI], const __bf16* Wp, long plane_elems,
-                                                     const bf16x8 (&ops)[kRB][NCH][2], unsigned char* lds) {
-    WStream<NI> w;
-    w.init(Wp, plane_elems, 32 * NCH);
-    w.load(0);
-    __syncthreads();                                          // the previous layer is done with the W buffers
-    w.store(lds);
-    w.load(kCK);
-    __syncthreads();
+    const long r0 = 32 * first_block, left = R - r0 - 32 * G, block = first_block + G;
+    const int rows = left < 32 ? (int)left : 32;                   // of this half's block; none if <= 0
+    if (r0 + 64 > R) {
 #pragma unroll
-    for (int c = 0; c < NCH; c++) {
-        w.multiply(acc, lds + (c & 1) * WStream<NI>::kBufW, [&](int rb, int s) { return ops[rb][c][s]; });
-        w.store(lds + ((c + 1) & 1) * WStream<NI>::kBufW);
-        w.load((c + 2) * kCK);
-        __syncthreads();
+        for (int r = 0; r < 32; r++) v[r >> 2 & 1][4 * (r >> 3) + (r & 3)] = r < rows ? v[r >> 2 & 1][4 * (r >> 3) + (r & 3)] : 0.f;
     }
-}
-
-struct SegmentRuns {
-    int my_seg, nv, runs, second;
-    unsigned starts;
-};
-
-// sum over the rows of each segment of the bf16-rounded act(acc + bias): two partial slots per block of 32 rows,
-// runs strictly inside a block written to `out` directly (fp32 accumulation, scale applied there)
-template <int ACT, bool BIAS, int NI>
-__device__ __forceinline__ void row_sums(const floatx16 (&acc)[NI], const float* __restrict__ bias, bool row_live,
-                                         const SegmentRuns& sr, float* slice, float* __restrict__ slots, long block,
-                                         long n_blocks, float* __restrict__ out, float scale) {
-    constexpr int O = 32 * NI;
-    const int lane = threadIdx.x & 63, m = lane & 31, g = lane >> 5;
+    const int my_seg = seg[r0 + lane < R ? r0 + lane : R - 1], before = __shfl_up(my_seg, 1);
+    const unsigned long long starts = __ballot(m > 0 && my_seg != before);
+    float* const slot = slots + (block < n_blocks ? block : 0) * O + col;
+    float* to = slot;                                              // of a block's first run; later ones lie inside the block
+    float sum = 0.f;
 #pragma unroll
-    for (int pass = 0; pass < NI / 2; pass++) {
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int ni = 2 * pass + h;
-#pragma unroll
-            for (int qq = 0; qq < 4; qq++) {
-                const float4 b = BIAS ? *reinterpret_cast<const float4*>(bias + 32 * ni + 8 * qq + 4 * g)
-                                      : make_float4(0.f, 0.f, 0.f, 0.f);
-                float4 v;
-                float* vp = &v.x;
-#pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    const float x = activate_c<ACT>(acc[ni][4 * qq + t] + (&b.x)[t]);
-                    vp[t] = row_live ? (float)(__bf16)x : 0.f;
-                }
-                *reinterpret_cast<float4*>(slice + m * kRed + 32 * h + 8 * qq + 4 * g) = v;
+    for (int r = 0; r < 32; r++) {
+        if (r > 0 && (starts >> r & 0x100000001ull)) {
+            const int s_lo = __builtin_amdgcn_readlane(my_seg, r), s_hi = __builtin_amdgcn_readlane(my_seg, 32 + r);
+            if (starts >> (r + 32 * G) & 1) {                      // (never at a row past the end: those repeat the last one)
+                *to = sum;
+                sum = 0.f;
+                to = out + (long)(G ? s_hi : s_lo) * O + col;
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const int col = 64 * pass + lane;
-        auto flush = [&](float sum, int run_start, int r) {
-            if (run_start == 0) {
-                slots[block * O + col] = sum;
-            } else if (r == 31) {
-                slots[(n_blocks + block) * O + col] = sum;
-            } else {
-                const long s_id = __shfl(sr.my_seg, r);
-                out[s_id * O + col] = scale * sum;
-            }
-        };
-        if (sr.nv > 0) {
-            if (sr.runs <= 2) {
-                float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-                for (int r = 0; r < 32; r++) {
-                    const float val = slice[r * kRed + lane];
-                    s0 += r < sr.second ? val : 0.f;
-                    s1 += r < sr.second ? 0.f : val;
-                }
-                flush(s0, 0, sr.second - 1);
-                if (sr.runs == 2) flush(s1, sr.second, sr.nv - 1);
-            } else {
-                float sum = 0.f;
-                int run_start = 0;
-                for (int r = 0; r < sr.nv; r++) {
-                    sum += slice[r * kRed + lane];
-                    if ((r == sr.nv - 1) || ((sr.starts >> (r + 1)) & 1u)) {
-                        flush(sum, run_start, r);
-                        sum = 0.f;
-                        run_start = r + 1;
-                    }
-                }
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        sum += v[r >> 2 & 1][4 * (r >> 3) + (r & 3)];
     }
+    if (rows <= 0) return;
+    if (to != slot && rows == 32) to = slots + (n_blocks + block) * O + col;
+    *to = sum;
 }
 
-template <int ACT>
-__global__ void __launch_bounds__(kThreads)
+template <int ACT, bool Y_PLANES>
+__global__ void __launch_bounds__(kThreads, 4)
 mlp_chain_bf16_kernel(const __bf16* __restrict__ X, long R, int I, const __bf16* __restrict__ Wa, long plane_a,
-                      const __bf16* __restrict__ Wb, long plane_b, const float* __restrict__ bias_b,
-                      const __bf16* __restrict__ Wc, long plane_c, const float* __restrict__ bias_c,
-                      const int* __restrict__ seg, float* __restrict__ slots_x, float* __restrict__ slots_h,
-                      long n_blocks, float* __restrict__ out_x, float* __restrict__ out_h, long tiles_total) {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[kLdsBytes];
-    static_assert(kLdsBytes / kWaves / 4 >= 32 * kRed, "a reduction pass needs 32 rows x 64 columns per wave");
+                      const __bf16* __restrict__ Wb, const float* __restrict__ bias_b, const __bf16* __restrict__ Wc,
+                      const float* __restrict__ bias_c, const int* __restrict__ seg, float* __restrict__ slots_x,
+                      float* __restrict__ slots_h, long n_blocks, float* __restrict__ out_x, float* __restrict__ out_h,
+                      long tiles_total) {
+    __shared__ __attribute__((aligned(16))) __bf16 lds[2 * kStageElems];
+    static_assert(kRows * kH == 2 * kStageElems && kRows * kD == kStageElems, "the layers' places");
 
     const long bid = blockIdx.x;
     const long per_xcd = (tiles_total + 7) / 8;
     const long tile = (bid % 8) * per_xcd + bid / 8;
     if (tile >= tiles_total) return;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int m = lane & 31, g = lane >> 5;
-    const long block0 = (tile * kWaves + wave) * kRB;         // this wave's first block of 32 rows
-    long ld_row[kRB];
-    bool row_live[kRB];
-    SegmentRuns sr[kRB];
-#pragma unroll
-    for (int rb = 0; rb < kRB; rb++) {
-        const long my_row = (block0 + rb) * 32 + m;
-        ld_row[rb] = my_row < R ? my_row : R - 1;
-        row_live[rb] = my_row < R;
-        sr[rb].my_seg = seg[ld_row[rb]];
-        const long rows_left = R - (block0 + rb) * 32;
-        sr[rb].nv = rows_left >= 32 ? 32 : (rows_left > 0 ? (int)rows_left : 0);
-        const int prev = __shfl_up(sr[rb].my_seg, 1);
-        sr[rb].starts = (unsigned)__ballot(g == 0 && (m == 0 || sr[rb].my_seg != prev));
-        sr[rb].runs = __popc(sr[rb].starts);
-        sr[rb].second = sr[rb].runs >= 2 ? __ffs(sr[rb].starts & ~1u) - 1 : 32;
-    }
-    float* slice = reinterpret_cast<float*>(lds) + wave * (kLdsBytes / kWaves / 4);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m = lane & 31, G = lane >> 5;
+    const long block0 = tile * kBlocks;
 
-    // ---- layer A: psi = Y x, x from memory (the lane's 16 bf16 of its row per chunk, two chunks ahead)
-    floatx16 acc_a[kRB][kD / 32];
-#pragma unroll
-    for (int rb = 0; rb < kRB; rb++)
-#pragma unroll
-        for (int ni = 0; ni < kD / 32; ni++)
-#pragma unroll
-            for (int q = 0; q < 16; q++) acc_a[rb][ni][q] = 0.f;
+    // ---- psi = Y x: wave = 32 columns of two row blocks; x by stages of 128 k, the next one in registers
+    const int cb = wave & 3, half = wave >> 2;
     {
-        using WS = WStream<kD / 32>;
-        WS w;
-        w.init(Wa, plane_a, I);
-        const int k_last = I - kCK;
-        auto load_x = [&](bf16x8 (&x)[kRB][2], int k0) {
-            k0 = k0 < I ? k0 : k_last;
+        Product<2, true, Y_PLANES> y;
+        y.start(Wa, plane_a, cb, I);
+        // a quarter of a row's pieces of 8 k to a thread; two rows of eight threads are four apart (fragment_at)
+        const int row = (tid >> 2 & 0x78) + (tid >> 2 & 1) * 4 + (tid >> 3 & 3);
+        const long my_row = block0 * 32 + row;
+        const __bf16* from = X + (my_row < R ? my_row : R - 1) * I + 8 * (tid & 3);
+        __bf16* to = lds + (row >> 5) * kStageBlock + fragment_at(row & 31, 8 * (tid & 3));
+        bf16x8 piece[4];
+        auto load = [&](int k0) {                                  // chunk j of the stage (past the end: the last one again)
 #pragma unroll
-            for (int rb = 0; rb < kRB; rb++) {
-                const __bf16* xrow = X + ld_row[rb] * I + 16 * g + k0;
-                x[rb][0] = *reinterpret_cast<const bf16x8*>(xrow);
-                x[rb][1] = *reinterpret_cast<const bf16x8*>(xrow + 8);
-            }
+            for (int j = 0; j < 4; j++) piece[j] = *reinterpret_cast<const bf16x8*>(from + (k0 + 32 * j < I ? k0 + 32 * j : I - 32));
         };
-        const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-        bf16x8 x0[kRB][2], x1[kRB][2];
-        w.load(0);
-        load_x(x0, 0);
-        w.store(lds);
-        w.load(kCK);
-        load_x(x1, kCK);
-        __syncthreads();
-        for (int k0 = 0; k0 < I; k0 += 2 * kCK) {
-            w.multiply(acc_a, lds, [&](int rb, int s) { return x0[rb][s]; });
-            w.store(lds + WS::kBufW);
-            __builtin_amdgcn_sched_barrier(0);
-            w.load(k0 + 2 * kCK);
-            __builtin_amdgcn_sched_barrier(0);
-            load_x(x0, k0 + 2 * kCK);
-            __syncthreads();
-            if (k0 + kCK >= I) {                              // a surplus odd chunk contributes nothing
+        load(0);
+        for (int k0 = 0, at = 0; k0 < I; k0 += kStage, at = kStageElems - at) {
 #pragma unroll
-                for (int rb = 0; rb < kRB; rb++) { x1[rb][0] = zero; x1[rb][1] = zero; }
-            }
-            w.multiply(acc_a, lds + WS::kBufW, [&](int rb, int s) { return x1[rb][s]; });
-            w.store(lds);
-            __builtin_amdgcn_sched_barrier(0);
-            w.load(k0 + 3 * kCK);
-            __builtin_amdgcn_sched_barrier(0);
-            load_x(x1, k0 + 3 * kCK);
+            for (int j = 0; j < 4; j++) *reinterpret_cast<bf16x8*>(to + at + 1024 * j) = piece[j];
+            if (k0 + kStage < I) load(k0 + kStage);
             __syncthreads();
+            const int left = I - k0;
+            y.run(lds + at + 2 * half * kStageBlock, kStageBlock, (left < kStage ? left : kStage) / 16);
+        }
+        __syncthreads();                                           // (the last stage may lie where psi goes)
+        __bf16* psi[4];                                            // of rows q % 4
+#pragma unroll
+        for (int i = 0; i < 4; i++) psi[i] = lds + 2 * half * kStageBlock + fragment_at(4 * G + i, 32 * cb + m);
+        float v[2][16];
+#pragma unroll
+        for (int mi = 0; mi < 2; mi++)
+#pragma unroll
+            for (int q = 0; q < 16; q++) {
+                const __bf16 r = (__bf16)y.acc[mi][q];
+                psi[q % 4][mi * kStageBlock + 64 * (q / 4)] = r;
+                v[mi][q] = (float)r;
+            }
+        sum_segments(v, block0 + 2 * half, R, seg, kD, 32 * cb + m, slots_x, n_blocks, out_x);
+    }
+    __syncthreads();
+
+    // ---- h1 = act(W1 psi + b1): wave = 32 columns of all rows
+    {
+        Product<kBlocks, false> h;
+        h.start(Wb, 0, wave, kD);
+        h.run(lds, kStageBlock, kD / 16);
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const int col = 32 * wave + 8 * t + 4 * G;
+            float b[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) b[i] = bias_b[col + i];
+#pragma unroll
+            for (int mi = 0; mi < kBlocks; mi++) {
+                bf16x4 v;
+#pragma unroll
+                for (int i = 0; i < 4; i++) v[i] = (__bf16)activate_c<ACT>(h.acc[mi][4 * t + i] + b[i]);
+                *reinterpret_cast<bf16x4*>(lds + mi * 32 * kH + fragment_at(m, col)) = v;
+            }
         }
     }
-    // sums of bf16(psi) per node, and psi as the operands of layer B
-    bf16x8 ops_a[kRB][kD / 32][2];
-#pragma unroll
-    for (int rb = 0; rb < kRB; rb++)
-        row_sums<0, false>(acc_a[rb], nullptr, row_live[rb], sr[rb], slice, slots_x, block0 + rb, n_blocks, out_x, 1.0f);
-    to_operands<0, false>(acc_a, nullptr, ops_a);
+    __syncthreads();
 
-    // ---- layer B: h1 = act(W1 psi + b1)
-    floatx16 acc_b[kRB][kH / 32];
+    // ---- h2 = act(W2 h1 + b2), only its sums per node leave the kernel
+    Product<kBlocks, true> h;
+    h.start(Wc, 0, wave, kH);
+    h.run(lds, 32 * kH, kH / 16);
+    const int col = 32 * wave + m;
+    const float b = bias_c[col];
 #pragma unroll
-    for (int rb = 0; rb < kRB; rb++)
+    for (int pair = 0; pair < kBlocks; pair += 2) {
+        float v[2][16];
 #pragma unroll
-        for (int ni = 0; ni < kH / 32; ni++)
+        for (int mi = 0; mi < 2; mi++)
 #pragma unroll
-            for (int q = 0; q < 16; q++) acc_b[rb][ni][q] = 0.f;
-    layer_from_registers<kH / 32, kD / 32>(acc_b, Wb, plane_b, ops_a, lds);
-    bf16x8 ops_b[kRB][kH / 32][2];
-    to_operands<ACT, true>(acc_b, bias_b, ops_b);
-
-    // ---- layer C: h2 = act(W2 h1 + b2), only its sums per node leave the kernel
-#pragma unroll
-    for (int rb = 0; rb < kRB; rb++)
-#pragma unroll
-        for (int ni = 0; ni < kH / 32; ni++)
-#pragma unroll
-            for (int q = 0; q < 16; q++) acc_b[rb][ni][q] = 0.f;
-    layer_from_registers<kH / 32, kH / 32>(acc_b, Wc, plane_c, ops_b, lds);
-#pragma unroll
-    for (int rb = 0; rb < kRB; rb++)
-        row_sums<ACT, true>(acc_b[rb], bias_c, row_live[rb], sr[rb], slice, slots_h, block0 + rb, n_blocks, out_h, 1.0f);
+            for (int q = 0; q < 16; q++) v[mi][q] = (float)(__bf16)activate_c<ACT>(h.acc[pair + mi][q] + b);
+        sum_segments(v, block0 + pair, R, seg, kH, col, slots_h, n_blocks, out_h);
+    }
 }
 
 }  // namespace
@@ -330,11 +285,14 @@ mlp_chain_bf16_kernel(const __bf16* __restrict__ X, long R, int I, const __bf16*
 
 using namespace mg;
 
+// fragments of W1, W2 and, where it is no wider than kPackedDimIn, Y
+static long chain_weight_elems(int dim_in) { return 2L * kH * kD + 2L * kH * kH + (dim_in <= kPackedDimIn ? 2L * kD * dim_in : 0); }
+
 extern "C" {
 
 int mg_mlp_chain_bf16_workspace_bytes(long rows, size_t* bytes) {
     MG_REQUIRE(bytes != nullptr && rows >= 0, "mg_mlp_chain_bf16_workspace_bytes: bad argument");
-    *bytes = (size_t)(2L * (ceil_div(rows, 32) + 1) * (kD + kH)) * sizeof(float);
+    *bytes = (size_t)(2L * (ceil_div(rows, 32) + 1) * (kD + kH)) * sizeof(float) + chain_weight_elems(kPackedDimIn) * sizeof(__bf16);
     return MG_OK;
 }
 
@@ -351,24 +309,32 @@ int mg_mlp_chain_bf16(const void* x, long rows, int dim_in, const void* packed_Y
                "mg_mlp_chain_bf16: null or unaligned operand");
     hipStream_t st = (hipStream_t)stream;
     const long n_blocks = ceil_div(rows, 32);
-    float* slots_x = static_cast<float*>(workspace);
+    __bf16* const w1 = static_cast<__bf16*>(workspace);
+    __bf16* const w2 = w1 + 2L * kH * kD;
+    __bf16* const y = w2 + 2L * kH * kH;
+    float* slots_x = reinterpret_cast<float*>(w1 + chain_weight_elems(kPackedDimIn));
     float* slots_h = slots_x + 2L * (n_blocks + 1) * kD;
     if (rows > 0) {
-        MG_REQUIRE(x && seg && aligned16(x), "mg_mlp_chain_bf16: null or unaligned row operand");
-        const long tiles = ceil_div(rows, 32 * kWaves);
+        MG_REQUIRE(x && seg && b1 && b2 && aligned16(x), "mg_mlp_chain_bf16: null or unaligned row operand");
+        const long tiles = ceil_div(rows, kRows);
         const long grid = ceil_div(tiles, 8) * 8;
         MG_REQUIRE(grid <= 0x7fffffffL, "mg_mlp_chain_bf16: grid too large");
-        // packed weights: planes of ceil(dim_out / 128) * 128 rows
-        const long plane_a = (long)kD * dim_in, plane_b = (long)kH * kD, plane_c = (long)kH * kH;
-#define MG_CHAIN_LAUNCH(A)                                                                                          \
-    hipLaunchKernelGGL((mlp_chain_bf16_kernel<A>), dim3((unsigned)grid), dim3(kThreads), 0, st,                        \
-                       static_cast<const __bf16*>(x), rows, dim_in, static_cast<const __bf16*>(packed_Y), plane_a,    \
-                       static_cast<const __bf16*>(packed_W1), plane_b, b1, static_cast<const __bf16*>(packed_W2),     \
-                       plane_c, b2, seg, slots_x, slots_h, n_blocks, sum_psi, sum_h2, tiles)
-        if (act == 1) MG_CHAIN_LAUNCH(1);
-        else if (act == 2) MG_CHAIN_LAUNCH(2);
-        else MG_CHAIN_LAUNCH(0);
-#undef MG_CHAIN_LAUNCH
+        // packed weights: planes of ceil(dim_out / 128) * 128 rows.  Their fragments are formed on every call: 4 us
+        const bool planes = dim_in > kPackedDimIn;
+        const __bf16 *from_y = static_cast<const __bf16*>(packed_Y), *from_1 = static_cast<const __bf16*>(packed_W1),
+                     *from_2 = static_cast<const __bf16*>(packed_W2);
+        const RepackAll all{{{from_1, (long)kH * kD, kH, kD, 1, w1}, {from_2, (long)kH * kH, kH, kH, 1, w2}, {from_y, (long)kD * dim_in, kD, dim_in, 0, y}}};
+        const long most = planes || dim_in < 2 * kH ? (long)kH * kH / 4 : (long)kD * dim_in / 4;
+        mlp_chain_repack_kernel<<<dim3((unsigned)ceil_div(most, 256), planes ? 2 : 3), dim3(256), 0, st>>>(all);
+        if (int code = check_launch("mlp_chain_repack_kernel")) return code;
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kThreads), 0, st, static_cast<const __bf16*>(x), rows, dim_in,
+                               planes ? from_y : y, (long)kD * dim_in, w1, b1, w2, b2, seg, slots_x, slots_h, n_blocks, sum_psi,
+                               sum_h2, tiles);
+        };
+        if (act == 1) planes ? launch(mlp_chain_bf16_kernel<1, true>) : launch(mlp_chain_bf16_kernel<1, false>);
+        else if (act == 2) planes ? launch(mlp_chain_bf16_kernel<2, true>) : launch(mlp_chain_bf16_kernel<2, false>);
+        else planes ? launch(mlp_chain_bf16_kernel<0, true>) : launch(mlp_chain_bf16_kernel<0, false>);
         if (int code = check_launch("mlp_chain_bf16_kernel")) return code;
     }
     rowsum_finish_kernel<<<dim3((unsigned)ceil_div(n_out * (kD / 4), 256)), dim3(256), 0, st>>>(

@@ -320,6 +320,29 @@ def test_scalar_message_chain_in_one_kernel(ops, kind, dim_in):
     assert not bool(s_psi[empty].any()) and not bool(s_h[empty].any())
 
 
+@pytest.mark.parametrize("rows,dim_in", [(1, 32), (127, 160), (129, 128), (261, 1024), (300, 1056)])
+def test_scalar_message_chain_at_the_edges_of_its_tiles(ops, rows, dim_in):
+    """Row counts beside the 128 rows of a workgroup, widths beside the 128 k of x that wait in LDS, and a Y on either side of
+    1024, the widest whose fragments the workspace holds (beyond, it is read from its planes).  psi in the order of the plain
+    kernel; bounds of the test above."""
+    g = torch.Generator().manual_seed(rows)
+    n_seg = 7
+    seg = torch.sort(torch.randint(0, n_seg, (rows,), generator=g)).values
+    x = torch.randn(rows, dim_in, generator=g).cuda().to(torch.bfloat16)
+    Y = (torch.randn(128, dim_in, generator=g) / dim_in ** 0.5).cuda()
+    W1, W2 = (torch.randn(256, 128, generator=g) / 128 ** 0.5).cuda(), (torch.randn(256, 256, generator=g) / 16).cuda()
+    b1, b2 = torch.randn(256, generator=g).cuda(), torch.randn(256, generator=g).cuda()
+    segc = seg.int().cuda()
+    s_psi, s_h = ops.mlp_chain_bf16(Y, x, W1, b1, W2, b2, ops.segment_row_ptr(segc, n_seg), segc, n_seg)
+    psi = ops.tensor_linear_bf16(Y, x)
+    h2 = ops.tensor_linear_bf16(W2, ops.tensor_linear_bf16(W1, psi, bias=b1, act=ops.ACT_LEAKY), bias=b2, act=ops.ACT_LEAKY)
+    ref_psi = torch.zeros(n_seg, 128, dtype=torch.float64).index_add_(0, seg, psi.double().cpu())
+    ref_h = torch.zeros(n_seg, 256, dtype=torch.float64).index_add_(0, seg, h2.double().cpu())
+    torch.testing.assert_close(s_psi.cpu().double(), ref_psi, rtol=1e-5, atol=2e-6 * float(ref_psi.abs().max()))
+    err = (s_h.cpu().double() - ref_h).abs()
+    assert float(err.max()) <= 2 * 2.0 ** -8 * float(h2.float().abs().max()) + 1e-5 * float(ref_h.abs().max())
+
+
 def test_messages_bf16_chain_equals_separate_kernels(pkg, ops):
     """messages_forward with the one-kernel scalar chain against the same call with the separate kernels."""
     bl = importlib.import_module("learned-dynamics_amd.bee_layers")
