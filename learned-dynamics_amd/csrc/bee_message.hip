@@ -19,7 +19,7 @@
 //
 // With Y2F the rank-2 sums do not leave the kernel either: the four waves of a workgroup hold the sums of
 // 4 / chunks whole nodes, the bias-free output linear of the rank-2 channel (K = 5 chan, dim_d <= 16 outputs) is
-// applied to them on the fp32 matrix cores (v_mfma_f32_16x16x4_f32: rows = the 9 components, 80 steps per wave),
+// applied to them (rank2_linear.hpp),
 // the waves' partial results are summed through LDS, and (node, dim_d, 9) is stored instead of (node, 9, 5, chan):
 // 45 chan floats per node less to write, the same again less to read, and one GEMM launch less.
 //
@@ -84,24 +84,9 @@ __global__ void __launch_bounds__(256) bee_geometry_kernel(const float* __restri
     rhat[3 * e + 2] = sz / len;
 }
 
-// max over the wave of non-negative values (NaN counts as zero), valid in lane 63: six cross-lane VALU operations (shifts within
-// rows of 16 lanes, then row broadcasts), no LDS traffic.  Such floats are ordered as their bits are, and an integer maximum
-// takes the moved operand directly: as fmaxf each step was a move, a shift, a canonicalisation and the maximum.
-__device__ __forceinline__ float wave_max_nonneg_last_lane(float v) {
-    auto step = [](unsigned x, auto ctrl, auto row_mask) {
-        const unsigned moved = (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, decltype(row_mask)::value, 0xf, false);
-        return x > moved ? x : moved;
-    };
-    unsigned x = __float_as_uint(fmaxf(v, 0.f));
-    x = step(x, std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});   // row_shr:1
-    x = step(x, std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});   // row_shr:2
-    x = step(x, std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});   // row_shr:4
-    x = step(x, std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});   // row_shr:8
-    x = step(x, std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});   // row_bcast:15
-    x = step(x, std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});   // row_bcast:31
-    return __uint_as_float(x);
+__device__ __forceinline__ float of_last_lane(float v) {
+    return __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(v), kWave - 1));
 }
-
 __device__ __forceinline__ long uniform(long v) {
     // the value is the same in every lane: keep it in scalar registers
     const int lo = __builtin_amdgcn_readfirstlane((int)(v & 0xffffffffL));
@@ -138,6 +123,7 @@ struct MessageArgs {
     int dim_d;
     float* out_d;
     int out_d_accumulate;
+    int split;                                                // the rank-2 linear may take fp16 pieces
 };
 
 // largest |sum| of a (node, channel): with the other channels of a chunk a row bound for the GEMMs that read S1 / S2
@@ -363,14 +349,14 @@ bee_message_kernel(const MessageArgs<T> g) {
                 for (int k = 0; k < 45; k++) put_row(o2, lane_bytes, k * row_bytes, (T)s2[k]);
             }
         }
-        if (g.node_max) {
+        if (Y2F || g.node_max) {
             const float mx = wave_max_nonneg_last_lane(active ? largest(s1, s2) : 0.f);
-            if (lane == kWave - 1 && valid) g.node_max[node * chunks + chunk] = mx;
-        }
-        if constexpr (Y2F) {
-            __shared__ __attribute__((aligned(16))) float lds[4 * kRank2Share];
-            rank2_linear_of_node_sums<>(s2, lds, chunk, chunks, valid, g.y2_packed, g.dim_d, g.out_d + node * (long)g.dim_d * 9,
-                                         g.out_d_accumulate != 0);
+            if (g.node_max && lane == kWave - 1 && valid) g.node_max[node * chunks + chunk] = mx;
+            if constexpr (Y2F) {
+                __shared__ __attribute__((aligned(16))) float lds[4 * kRank2Share];
+                rank2_linear_of_node_sums<>(s2, of_last_lane(mx), g.split != 0, lds, chunk, chunks, valid, g.y2_packed, g.dim_d,
+                                            g.out_d + node * (long)g.dim_d * 9, g.out_d_accumulate != 0);
+            }
         }
     }
 }
@@ -418,12 +404,6 @@ __device__ __forceinline__ void wait_for_edge(int k, int after) {
         wait_vmcnt<0>();
     }
 }
-// a value that is uniform over the wave and never written while the kernel runs: a scalar load also beside the asm above
-template <typename V>
-__device__ __forceinline__ V scalar_at(const V* p) {
-    return *(const __attribute__((address_space(4))) V*)(unsigned long)p;
-}
-
 // EMAX: the edges' maxima are asked for.  Y2F: as above.
 template <typename T, bool EMAX, bool Y2F>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 5, sizeof(T) == 4 ? 4 : 5)))
@@ -546,29 +526,68 @@ bee_message_ring_kernel(const MessageArgs<T> g) {
 #pragma unroll
                 for (int k = 0; k < 45; k++) put_row(o2, lane_bytes, k * row_bytes, (T)s2[k]);
             }
-            if (g.node_max) {
-                const float mx = wave_max_nonneg_last_lane(largest(s1, s2));
-                if (lane == kWave - 1) g.node_max[node * chunks + chunk] = mx;
-            }
         }
-        if constexpr (Y2F)
-            rank2_linear_of_node_sums<kShare / 4>(s2, reinterpret_cast<float*>(lds), chunk, chunks, valid, g.y2_packed, g.dim_d,
-                                                  g.out_d + node * (long)g.dim_d * 9, g.out_d_accumulate != 0);
+        if (Y2F || g.node_max) {
+            const float mx = wave_max_nonneg_last_lane(largest(s1, s2));
+            if (g.node_max && lane == kWave - 1 && valid) g.node_max[node * chunks + chunk] = mx;
+            if constexpr (Y2F)
+                rank2_linear_of_node_sums<kShare / 4>(s2, of_last_lane(mx), g.split != 0, reinterpret_cast<float*>(lds), chunk, chunks, valid,
+                                                      g.y2_packed, g.dim_d, g.out_d + node * (long)g.dim_d * 9, g.out_d_accumulate != 0);
+        }
     }
 }
 
-// Y2 (dim_d, 5 chan), row stride ld -> [chunk][label][tq][lane = 16 kk + j][tr] = Y2[j][label chan + 64 chunk + 16 kk + 4 tq + tr]
-// (zero for j >= dim_d): what lane (kk, j) of the fused kernel multiplies in steps 4 tq .. 4 tq + 3 of a label
+// The inverse scales of the 16 outputs of a rank-2 weight, one workgroup each
+__global__ void __launch_bounds__(256) rank2_weight_scales_kernel(const float* __restrict__ Y2, long ld, int chan, int dim_d,
+                                                                  float* __restrict__ inv) {
+    __shared__ float part[4];
+    __shared__ int odd;
+    const int j = blockIdx.x;
+    if (threadIdx.x == 0) odd = 0;
+    __syncthreads();
+    float mx = 0.f;
+    for (int k = threadIdx.x; j < dim_d && k < 5 * chan; k += 256) {
+        const float v = fabsf(Y2[j * ld + k]);
+        if (v < __builtin_inff()) mx = fmaxf(mx, v);
+        else odd = 1;
+    }
+    mx = wave_max_nonneg_last_lane(mx);
+    if ((threadIdx.x & 63) == 63) part[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float one;
+        pow2_scale(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])), &one);
+        inv[j] = odd ? mark_weight(one) : one;
+    }
+}
+// Y2 (dim_d, 5 chan), row stride ld, into the order of rank2_linear.hpp: threads below 5120 chunks one fp32 value each, those behind
+// them eight pieces
 __global__ void __launch_bounds__(256) pack_rank2_weight_kernel(const float* __restrict__ Y2, long ld, int chan,
                                                                 int dim_d, float* __restrict__ packed) {
     const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long total = (long)(chan / 64) * 5 * 4 * 64 * 4;
-    if (idx >= total) return;
-    const int tr = (int)(idx & 3), lane = (int)((idx >> 2) & 63), tq = (int)((idx >> 8) & 3);
-    const long rest = idx >> 10;                              // chunk * 5 + label
-    const int label = (int)(rest % 5), chunk = (int)(rest / 5);
-    const int j = lane & 15, kk = lane >> 4;
-    packed[idx] = j < dim_d ? Y2[j * ld + (long)label * chan + 64 * chunk + 16 * kk + 4 * tq + tr] : 0.f;
+    const int chunks = chan / 64;
+    const long plain = (long)chunks * kRank2Fp32;
+    const int lane = (int)(idx < plain ? idx >> 2 : idx) & 63, j = lane & 15, kk = lane >> 4;
+    auto weight = [&](int chunk, int label, int c) { return j < dim_d ? Y2[j * ld + (long)label * chan + 64 * chunk + 16 * kk + c] : 0.f; };
+    if (idx < plain) {
+        const int tr = (int)(idx & 3), tq = (int)((idx >> 8) & 3);
+        const long rest = idx >> 10;                          // chunk * 5 + label
+        packed[idx] = weight((int)(rest / 5), (int)(rest % 5), 4 * tq + tr);
+        return;
+    }
+    const long of = (idx - plain) >> 6;                       // chunk * 24 + fragment (plain is a multiple of 64)
+    if (of >= chunks * 24L) return;
+    const int chunk = (int)(of / 24), f = (int)(of % 24), t = (f >> 1) & 3;
+    _Float16* const pieces = reinterpret_cast<_Float16*>(packed + plain);
+    const float scale = 1.0f / unmark_weight(reinterpret_cast<const float*>(pieces + (long)chunks * kRank2Pieces)[j]);   // (a power of two)
+    halfx8 out;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const float v = weight(chunk, f < 16 ? 2 * (f >> 3) + (e & 1) : 4, 4 * t + (e >> 1)) * scale;
+        const _Float16 hi = (_Float16)v, lo = (_Float16)(v - (float)hi);
+        out[e] = (f & 1) ? lo : hi;
+    }
+    *reinterpret_cast<halfx8*>(pieces + (of * 64 + lane) * 8) = out;
 }
 
 }  // namespace
@@ -591,7 +610,7 @@ static int launch_bee_message(const char* what, const int* row_ptr, const int* d
     MG_REQUIRE((long)n_nodes * 9 * chan * (long)sizeof(T) < (1L << 32),
                "%s: the rank-2 node rows must stay below 4 GiB (32-bit row offsets)", what);
     const MessageArgs<T> args{row_ptr, dst, node_order, (long)n_nodes, rhat, enc, La, Lv, Ld, chan, enc_W, enc_b, P0, S1, S2,
-                              node_max, edge_max, y2_packed, dim_d, out_d, out_d_accumulate};
+                              node_max, edge_max, y2_packed, dim_d, out_d, out_d_accumulate, mg_get_linear_mode() == kLinearF16x2};
     // one item per wave, four per workgroup, an eighth of the items per XCD (the kernel's loop then makes one trip)
     auto launch = [&](auto kernel, long items) -> int {
         const long blocks = 8 * ceil_div(ceil_div(items, 8), 4);
@@ -646,14 +665,17 @@ int mg_bee_message_rank2_supported(int chan, int dim_d) { return rank2_fusable(c
 
 int mg_bee_rank2_weight_bytes(int chan, size_t* bytes) {
     MG_REQUIRE(bytes != nullptr && chan >= 0, "mg_bee_rank2_weight_bytes: bad argument");
-    *bytes = (size_t)ceil_div(chan, 64) * 5 * 4 * 64 * 4 * sizeof(float);
+    *bytes = rank2_weight_bytes(chan);
     return MG_OK;
 }
 
 int mg_bee_pack_rank2_weight(const float* Y2, long ld, int chan, int dim_d, float* packed, mg_stream_t stream) {
     MG_REQUIRE(rank2_fusable(chan, dim_d), "mg_bee_pack_rank2_weight: needs chan = 64, 128 or 256 and dim_d <= 16");
     MG_REQUIRE(Y2 && packed && ld >= 5L * chan, "mg_bee_pack_rank2_weight: null pointer or short rows");
-    const long total = (long)(chan / 64) * 5 * 4 * 64 * 4;
+    const long chunks = chan / 64, total = chunks * (kRank2Fp32 + kRank2Pieces / 8);
+    hipLaunchKernelGGL(rank2_weight_scales_kernel, dim3(16), dim3(256), 0, (hipStream_t)stream, Y2, ld, chan, dim_d,
+                       packed + chunks * (kRank2Fp32 + kRank2Pieces / 2));
+    if (int code = check_launch("rank2_weight_scales_kernel")) return code;
     hipLaunchKernelGGL(pack_rank2_weight_kernel, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, (hipStream_t)stream,
                        Y2, ld, chan, dim_d, packed);
     return check_launch("mg_bee_pack_rank2_weight");

@@ -200,10 +200,13 @@ __global__ void __launch_bounds__(256) node_products_grad_kernel(long n_nodes, i
 // in one pass: a wave owns (node, 64-channel chunk), a lane one channel; the 45 product values stay in registers
 // and go through rank2_linear_of_node_sums.  Reads the 26 operand rows of a node once (unit stride), writes
 // (node, dim_d, 9); the products themselves are never stored.  For chan = 64, 128 or 256 and dim_d <= 16.
-// (A persistent variant whose workgroups walk over the nodes with the next node's operands already requested was
-// measured at 65 536 nodes, 256 channels: 0.61 ms against 0.57 ms; the kernel is bound by the matrix instructions,
-// 0.31 ms of pipe time at 9 of 16 rows used, and what each wave does around them, not by the latency of its loads.)
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8)))
+// 256 channels, 16 outputs, x_d of 16 channels: 780 us at 65 536 nodes, 78 at 8192, 24 at 2048; with the linear on the fp32 matrix
+// cores, x_d through LDS (a broadcast read costs as much as any other) and the scalar and vector products stored before the linear 884, 98
+// and 29.  What bounds it: a wave's chain of loads (of 780 us the linear takes 330, the rank-2 operands 180, the stores 175, and 300 are left
+// without all three), beside 9 GB of weights from the L2.  A chunk's weights in LDS for eight nodes, the chunks of a node in
+// turn: 753 us, but 31 at 2048 nodes, and 1030 with the stores at the end of a chunk, for want of registers; five waves a SIMD 994 us
+// (35 spilled).
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
 node_rank2_linear_kernel(long n_nodes, int chan, const float* __restrict__ l0,
                                                                 const float* __restrict__ l1, const float* __restrict__ l2,
                                                                 const float* __restrict__ r0, const float* __restrict__ r1,
@@ -213,20 +216,26 @@ node_rank2_linear_kernel(long n_nodes, int chan, const float* __restrict__ l0,
                                                                 float* __restrict__ P1, float* __restrict__ node_max,
                                                                 const float* __restrict__ x_d,
                                                                 const float* __restrict__ L2t,
-                                                                const float* __restrict__ R2t, int dim_in2) {
+                                                                const float* __restrict__ R2t, int dim_in2, int split) {
     __shared__ __attribute__((aligned(16))) float rank2_lds[4 * kRank2Share];
-    __shared__ float xd_buf[4][16 * 9];
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int chunks = chan / kWave;
     const long items = n_nodes * chunks;
     long item = (long)blockIdx.x * 4 + wave;
     const bool valid = item < items;                           // uniform over the wave
     item = valid ? item : items - 1;
-    const long node = item / chunks;
-    const int chunk = (int)(item - node * chunks);
+    const long node = item >> (chunks >> 1);                   // (1, 2 or 4 of them)
+    const int chunk = (int)item & (chunks - 1);
     const int c = chunk * kWave + lane;
-    float s2[45];
+    float s2[45], bound = 0.f, lower[18];
     if (valid) {
+        // x_d is read as scalars below, some lines at a time: all of them are asked for here, beside the other operands
+        float touched[9];
+        if (x_d) {
+            const float* src = x_d + node * (long)(dim_in2 * 9);
+#pragma unroll
+            for (int t = 0; t < 9; t++) touched[t] = scalar_at(src + (16 * t < dim_in2 * 9 ? 16 * t : dim_in2 * 9 - 1));
+        }
         const float a = l0[node * chan + c], b = r0[node * chan + c];
         float u[3], v[3], L[9], R[9];
 #pragma unroll
@@ -236,24 +245,43 @@ node_rank2_linear_kernel(long n_nodes, int chan, const float* __restrict__ l0,
         }
         if (x_d) {
             // the rank-2 operands are formed here: l2[k] = sum_i L2[c, i] x_d[node, i, k] (dim_in2 <= 16 input
-            // channels; the node's 9 dim_in2 values go through LDS and are read back as broadcasts, the weights come
+            // channels; the node's 9 dim_in2 values are scalars of the wave, the weights come
             // transposed, (dim_in2, chan), one coalesced row per input channel).  Two GEMMs that would each write
             // (node, 9, chan) and this kernel's read of both are not needed.
-            float* xd = xd_buf[wave];
             const float* src = x_d + node * (long)(dim_in2 * 9);
-            for (int t = lane; t < dim_in2 * 9; t += kWave) xd[t] = src[t];
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
             for (int k = 0; k < 9; k++) { L[k] = 0.f; R[k] = 0.f; }
-            for (int i = 0; i < dim_in2; i++) {
-                const float wl = L2t[(long)i * chan + c], wr = R2t[(long)i * chan + c];
+            // four input channels at a time, the weights of the next four requested before these are used (past the end: the last one's)
+            float wl[4], wr[4];
+            auto weights = [&](int i0) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int i = i0 + j < dim_in2 ? i0 + j : dim_in2 - 1;
+                    wl[j] = L2t[(long)i * chan + c];
+                    wr[j] = R2t[(long)i * chan + c];
+                }
+            };
+            auto add = [&](int i, float w_l, float w_r) {
 #pragma unroll
                 for (int k = 0; k < 9; k++) {
-                    const float xv = xd[i * 9 + k];
-                    L[k] = fmaf(wl, xv, L[k]);
-                    R[k] = fmaf(wr, xv, R[k]);
+                    const float xv = scalar_at(src + i * 9 + k);
+                    L[k] = fmaf(w_l, xv, L[k]);
+                    R[k] = fmaf(w_r, xv, R[k]);
+                }
+            };
+            weights(0);
+#pragma unroll
+            for (int t = 0; t < 9; t++) asm volatile("" ::"s"(touched[t]));
+            for (int i0 = 0; i0 < dim_in2; i0 += 4) {
+                const float l[4] = {wl[0], wl[1], wl[2], wl[3]}, r[4] = {wr[0], wr[1], wr[2], wr[3]};
+                weights(i0 + 4);
+                if (i0 + 4 <= dim_in2) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) add(i0 + j, l[j], r[j]);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 3; j++)
+                        if (i0 + j < dim_in2) add(i0 + j, l[j], r[j]);
                 }
             }
         } else {
@@ -263,37 +291,33 @@ node_rank2_linear_kernel(long n_nodes, int chan, const float* __restrict__ l0,
                 R[k] = r2[(node * 9 + k) * chan + c];
             }
         }
-        if (P0) {
-            // the scalar and vector products as well, stored in the layout of mg_bee_node_products with their
-            // maximum per (node, chunk): the operands are in registers once, and the two GEMMs that follow read
-            // 18 chan floats per node instead of gathering 26 chan through their operand loads
-            float dot = 0.f, ddot = 0.f;
+        // the scalar and vector products as well (stored below)
+        lower[0] = a * b;
+        lower[1] = u[0] * v[0] + u[1] * v[1] + u[2] * v[2];
+        lower[2] = 0.f;
 #pragma unroll
-            for (int x = 0; x < 3; x++) dot += u[x] * v[x];
+        for (int k = 0; k < 9; k++) lower[2] += L[k] * R[k];
+        const float cr[3] = {u[1] * v[2] - u[2] * v[1], u[2] * v[0] - u[0] * v[2], u[0] * v[1] - u[1] * v[0]};
 #pragma unroll
-            for (int k = 0; k < 9; k++) ddot += L[k] * R[k];
-            float* p0 = P0 + (node * 3) * chan + c;
-            __builtin_nontemporal_store(a * b, p0);
-            __builtin_nontemporal_store(dot, p0 + chan);
-            __builtin_nontemporal_store(ddot, p0 + 2 * chan);
-            float mx = fmaxf(fabsf(a * b), fmaxf(fabsf(dot), fabsf(ddot)));
-            const float cr[3] = {u[1] * v[2] - u[2] * v[1], u[2] * v[0] - u[0] * v[2], u[0] * v[1] - u[1] * v[0]};
-#pragma unroll
-            for (int x = 0; x < 3; x++) {
-                float* p1 = P1 + ((node * 3 + x) * 5) * chan + c;
-                const float q[5] = {a * v[x], u[x] * b, u[0] * R[3 * x] + u[1] * R[3 * x + 1] + u[2] * R[3 * x + 2],
-                                    L[3 * x] * v[0] + L[3 * x + 1] * v[1] + L[3 * x + 2] * v[2], cr[x]};   // 011 101 121 211 111
-#pragma unroll
-                for (int t = 0; t < 5; t++) {
-                    __builtin_nontemporal_store(q[t], p1 + t * chan);
-                    mx = fmaxf(mx, fabsf(q[t]));
-                }
-            }
-            if (node_max) {
-                for (int d = 1; d < kWave; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
-                if (lane == 0) node_max[node * chunks + chunk] = mx;
-            }
+        for (int x = 0; x < 3; x++) {                          // 011 101 121 211 111
+            lower[3 + 5 * x] = a * v[x];
+            lower[4 + 5 * x] = u[x] * b;
+            lower[5 + 5 * x] = u[0] * R[3 * x] + u[1] * R[3 * x + 1] + u[2] * R[3 * x + 2];
+            lower[6 + 5 * x] = L[3 * x] * v[0] + L[3 * x + 1] * v[1] + L[3 * x + 2] * v[2];
+            lower[7 + 5 * x] = cr[x];
         }
+        float ml = fabsf(a), mr = fabsf(b);
+#pragma unroll
+        for (int x = 0; x < 3; x++) {
+            ml = fmaxf(ml, fabsf(u[x]));
+            mr = fmaxf(mr, fabsf(v[x]));
+        }
+#pragma unroll
+        for (int k = 0; k < 9; k++) {
+            ml = fmaxf(ml, fabsf(L[k]));
+            mr = fmaxf(mr, fabsf(R[k]));
+        }
+        bound = 3.0f * ml * mr;                                // (three terms at most)
 #pragma unroll
         for (int x = 0; x < 3; x++) {
             // 212: row x of L crossed with v
@@ -312,8 +336,27 @@ node_rank2_linear_kernel(long n_nodes, int chan, const float* __restrict__ l0,
     } else {
 #pragma unroll
         for (int k = 0; k < 45; k++) s2[k] = 0.f;
+#pragma unroll
+        for (int k = 0; k < 18; k++) lower[k] = 0.f;
     }
-    rank2_linear_of_node_sums<>(s2, rank2_lds, chunk, chunks, valid, y2_packed, dim_d, out + node * (long)dim_d * 9);
+    bound = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(wave_max_nonneg_last_lane(bound)), kWave - 1));
+    rank2_linear_of_node_sums<>(s2, bound, split != 0, rank2_lds, chunk, chunks, valid, y2_packed, dim_d, out + node * (long)dim_d * 9);
+    if (P0 && valid) {
+        // In the layout of mg_bee_node_products with their maximum per (node, chunk): the operands are in registers once, and the
+        // two GEMMs that follow read 18 chan floats per node instead of gathering 26 chan through their operand loads.  Behind everything
+        // that loads: the queue of a wave completes in order, and a load behind these stores waits for memory to take them.
+        float mx = 0.f;
+#pragma unroll
+        for (int k = 0; k < 18; k++) {
+            float* to = k < 3 ? P0 + (node * 3 + k) * chan + c : P1 + (node * 15 + k - 3) * chan + c;
+            __builtin_nontemporal_store(lower[k], to);
+            mx = fmaxf(mx, fabsf(lower[k]));
+        }
+        if (node_max) {
+            mx = wave_max_nonneg_last_lane(mx);
+            if (lane == kWave - 1) node_max[node * chunks + chunk] = mx;
+        }
+    }
 }
 
 template <typename T>
@@ -376,7 +419,8 @@ int mg_bee_node_products_rank2(long n_nodes, int chan, const float* l0, const fl
     const long blocks = ceil_div(n_nodes * (chan / kWave), 4);
     MG_REQUIRE(blocks < (1L << 31), "mg_bee_node_products_rank2: too many nodes for one launch");
     hipLaunchKernelGGL(node_rank2_linear_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, n_nodes,
-                       chan, l0, l1, l2, r0, r1, r2, packed_Y2, dim_d, out_d, P0, P1, node_max, x_d, L2t, R2t, dim_in2);
+                       chan, l0, l1, l2, r0, r1, r2, packed_Y2, dim_d, out_d, P0, P1, node_max, x_d, L2t, R2t, dim_in2,
+                       mg_get_linear_mode() == kLinearF16x2);
     return check_launch("mg_bee_node_products_rank2");
 }
 

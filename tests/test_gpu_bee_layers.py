@@ -134,6 +134,48 @@ def test_bee_message_with_the_rank2_linear_inside(ops, chan, dim_d, N, E):
     assert_parity_of(out2, lambda dt: (s2.to(dt) @ Y2.cpu().to(dt).t()).transpose(1, 2), "after the weight changed")
 
 
+@pytest.mark.parametrize("chan,dim_d,N", [(256, 16, 9), (64, 3, 5), (128, 16, 3)])
+@pytest.mark.parametrize("what", ["plain", "infinity", "beyond the pieces", "odd weight"])
+def test_rank2_linear_in_pieces_and_in_fp32(ops, chan, dim_d, N, what):
+    """The rank-2 linear inside the edge and the node kernel takes fp16 pieces where they can carry a wave's values and an output's
+    weights, and fp32 products elsewhere (everywhere in mode 0): the same entries are finite in both modes, and those agree to
+    fp32 rounding, 2^-23 of sum |w| |p| (a bound of either's distance from exact: both sum fewer than 2^9 partial sums of one sign each)."""
+    g = torch.Generator().manual_seed(chan + N)
+    t = [torch.randn(N, *k, chan, generator=g) for k in ((), (3,), (9,), (), (3,), (9,))]
+    W = torch.randn(dim_d, 5 * chan, generator=g) / (5 * chan) ** 0.5
+    if what == "infinity":
+        t[2][1, 4, 7] = float("inf")
+        t[1][2, 0, chan - 1] = float("-inf")
+    elif what == "beyond the pieces":
+        t[1][1] *= 2.0 ** 55
+        t[2][1] *= 2.0 ** 55
+        t[5][1] *= 2.0 ** 50
+    elif what == "odd weight":
+        W[dim_d - 1, 3] = float("nan")
+    t, W = [x.cuda() for x in t], W.cuda()
+    E = 4 * N
+    row_ptr, dst = (torch.arange(N + 1) * 4).int().cuda(), torch.randint(0, N, (E,), generator=g).int().cuda()
+    enc, rhat = ops.bee_edge_geometry((torch.randn(E, 3, generator=g) * 2.5).cuda(), 6.0)
+    encW, encb = (torch.randn(chan, 8, generator=g) * 0.3).cuda(), torch.randn(chan, generator=g).cuda()
+
+    def run():
+        return (ops.bee_node_products_rank2(*t, W),
+                ops.bee_message(row_ptr, dst, rhat, enc, *t[:3], encW, encb, Y2=W)[2])
+    sums = (ops.bee_node_products(*t)[2], ops.bee_message(row_ptr, dst, rhat, enc, *t[:3], encW, encb)[2])
+    pieces = run()
+    mode = ops.get_linear_mode()
+    ops.set_linear_mode(ops.LINEAR_FP32_MFMA)
+    try:
+        plain = run()
+    finally:
+        ops.set_linear_mode(mode)
+    for y, z, p in zip(pieces, plain, sums):
+        finite = torch.isfinite(z)
+        assert torch.equal(torch.isfinite(y), finite) and bool(finite.any())
+        bound = (p.double().abs().reshape(N, 9, 5 * chan) @ W.double().abs().t()).transpose(1, 2)
+        assert bool(((y.double() - z.double()).abs() <= 2.0 ** -23 * bound)[finite].all())
+
+
 @pytest.mark.parametrize("chan,bf16", [(64, False), (128, False), (256, False), (64, True), (192, True)])
 def test_bee_message_rows_of_every_short_length(ops, chan, bf16):
     """Rows of 0 to 9 and of 33 edges, through LDS (16-byte aligned operands) and through registers (operands 4 bytes off): both do
