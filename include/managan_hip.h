@@ -973,6 +973,16 @@ int mg_group_norm(int mode, const float* x, long x_stride, const float* mul, lon
                   int batch, int nodes, int chan, int groups, int comps, float eps,
                   const float* gamma, const float* beta, const float* add, long add_stride,
                   const float* res, void* scratch, float* out, mg_stream_t stream);
+/* mg_group_norm in mode 0 of up to MG_TENS_NORMS dense tensors x (batch, nodes, chan, comps) of the same nodes in two launches, with res
+ * (or NULL) added.  scratch: the sum over the norms of mg_group_norm_scratch_bytes(batch, groups). */
+#define MG_TENS_NORMS 3
+typedef struct mg_tens_norm {
+    const float *x, *gamma, *res;
+    float* out;
+    int chan, comps, groups;
+    float eps;
+} mg_tens_norm;
+int mg_tens_group_norms(const mg_tens_norm* norms, int count, int batch, int nodes, void* scratch, mg_stream_t stream);
 /* Gradients of mode 0 for dense x and dy (batch, nodes, chan, comps), nothing added: dx like x, dgamma (chan).  scratch: what the
  * forward call of this x left there. */
 int mg_tensor_norm_grad_workspace_bytes(int batch, int chan, int groups, int comps, size_t* bytes /* host */);   /* any nodes */

@@ -112,6 +112,7 @@ _SIGNATURES = {
     "mg_tensor_norm_grad_workspace_bytes_of": [i32, i32, i32, i32, i32, ctypes.POINTER(ctypes.c_size_t)],
     "mg_tensor_norm_grad": [vp, vp, i32, i32, i32, i32, i32, f32, vp, vp, vp, vp, vp, vp],
     "mg_group_norm": [i32, vp, i64, vp, i64, i32, i32, i32, i32, i32, f32, vp, vp, vp, i64, vp, vp, vp, vp],
+    "mg_tens_group_norms": [vp, i32, i32, i32, vp, vp],
     "mg_tens_sigmoid": [i32, vp, i64, vp, vp],
     "mg_painn_update_maps_supported": [i32],
     "mg_painn_update_maps": [vp, vp, i64, i32, vp, vp, vp, vp, vp, vp],

@@ -197,8 +197,12 @@ class SelfTensProds(nn.Module):
         y_a = y_a.reshape(*rest, dim_a)
         y_v = y_v.reshape(*rest, dim_v, 3)
         y_d = y_d.reshape(*rest, dim_d, 3, 3)
+        res = (in_a.contiguous(), in_v.contiguous(), in_d.contiguous()) if residual else (None, None, None)
+        norms = (self.gn_a, self.gn_v, self.gn_d)
+        if len(rest) == 2 and all(diff.plain_call(gn, TensGroupNorm) for gn in norms):
+            return tuple(ops.tens_group_norms([(y, gn.groups, gn.gamma.reshape(-1).contiguous(), gn.epsilon, r)
+                                               for gn, y, r in zip(norms, (y_a, y_v, y_d), res)]))
         if residual:
-            res = (in_a.contiguous(), in_v.contiguous(), in_d.contiguous())
             return tuple(ops.concurrent([lambda: self.gn_a(y_a, res=res[0]), lambda: self.gn_v(y_v, res=res[1]),
                                          lambda: self.gn_d(y_d, res=res[2])], rows))
         return tuple(ops.concurrent([lambda: self.gn_a(y_a), lambda: self.gn_v(y_v), lambda: self.gn_d(y_d)], rows))

@@ -133,18 +133,15 @@ __device__ __forceinline__ float added(float y, float first, float second) {
 // 3 us on one system and 5 on 32 of them; each node array had one).
 // VEC: the vector output of a PaiNN Update, whose rows have as many channels, beside it (layout VEC - 1): 16 336 nodes of
 // 128 channels 22.5 us, 26.0 in two launches, 337 nodes 9.7, 9.6 and a launch.
-template <int VEC = 0>
-__global__ void __launch_bounds__(256) group_apply_kernel(const float* __restrict__ x, long x_stride,
-                                                          const float* __restrict__ mul, long mul_stride,
-                                                          const double* __restrict__ partial, int N, int chan,
-                                                          int groups, int T, int mode, float eps,
-                                                          const float* __restrict__ gamma, const float* __restrict__ beta,
-                                                          const float* __restrict__ add, long add_stride,
-                                                          const float* __restrict__ res, float* __restrict__ out,
-                                                          const UpdateVec vec) {
+template <int VEC>
+__device__ __forceinline__ void group_apply(const float* __restrict__ x, long x_stride, const float* __restrict__ mul, long mul_stride,
+                                            const double* __restrict__ partial, int N, int chan, int groups, int T, int mode, float eps,
+                                            const float* __restrict__ gamma, const float* __restrict__ beta,
+                                            const float* __restrict__ add, long add_stride, const float* __restrict__ res,
+                                            float* __restrict__ out, const UpdateVec& vec, int k_block) {
     __shared__ float2 stats[256];                                  // (a position a thread: no more groups than that)
     const int CT = chan * T, b = blockIdx.z, per = chan / groups * T;
-    const int k_first = blockIdx.x * blockDim.x, k = k_first + (int)threadIdx.x;
+    const int k_first = k_block * blockDim.x, k = k_first + (int)threadIdx.x;
     const int k_last = k_first + (int)blockDim.x < CT ? k_first + (int)blockDim.x - 1 : CT - 1, g_first = k_first / per;
     const bool live = k < CT;
     const long x_row = x_stride * T, m_row = mul_stride * T, a_row = add_stride * T;
@@ -182,6 +179,87 @@ __global__ void __launch_bounds__(256) group_apply_kernel(const float* __restric
                 if (node < N) update_vec<VEC - 1>(vec, (long)b * N + node, CT, k);
         }
     }
+}
+template <int VEC = 0>
+__global__ void __launch_bounds__(256) group_apply_kernel(const float* __restrict__ x, long x_stride,
+                                                          const float* __restrict__ mul, long mul_stride,
+                                                          const double* __restrict__ partial, int N, int chan,
+                                                          int groups, int T, int mode, float eps,
+                                                          const float* __restrict__ gamma, const float* __restrict__ beta,
+                                                          const float* __restrict__ add, long add_stride,
+                                                          const float* __restrict__ res, float* __restrict__ out,
+                                                          const UpdateVec vec) {
+    group_apply<VEC>(x, x_stride, mul, mul_stride, partial, N, chan, groups, T, mode, eps, gamma, beta, add, add_stride, res, out, vec, blockIdx.x);
+}
+
+// Several tensor norms of the same nodes (those of the three ranks) in the two launches of one.
+struct NormJob {
+    const float *x, *gamma, *res;
+    float* out;
+    double* partial;
+    int chan, groups, T, first_block;                              // of the apply kernel's grid
+    float eps;
+};
+struct NormJobs {
+    NormJob job[MG_TENS_NORMS];
+    int count;
+};
+// Sums of squares over a chunk's nodes (x), a box (y) and a job (z), for all groups at once: a thread keeps one position k = c T + t of
+// the rows (and a workgroup takes several rows at a time where they are shorter than it), whole rows are read, and the positions of a
+// group are added at the end (group_stats_kernel has a workgroup for every group as well, each with two reductions of its own).  The norms of
+// 256, 64 x 3 and 16 x 9 floats a node with a residual, in this pair of launches and one after the other: 32 boxes of 2048 nodes 119 and
+// 207 us, of 150 nodes 29 and 95, one box of 2048 15 and 51 with the host calls.  Bound by reading x twice and what is added once.
+__global__ void __launch_bounds__(256) tens_stats_kernel(const NormJobs jobs, int N) {
+    __shared__ double sums[256];
+    const NormJob& j = jobs.job[blockIdx.z];
+    const int chunk = blockIdx.x, b = blockIdx.y, CT = j.chan * j.T, per = j.chan / j.groups * j.T;
+    const int nodes = (N + kChunks - 1) / kChunks, n_lo = chunk * nodes, n_hi = n_lo + nodes < N ? n_lo + nodes : N;
+    const int across = CT < 256 ? CT : 256, down = 256 / across;   // positions of a row, rows at a time
+    const int sub = threadIdx.x / across, lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    double* const partial = j.partial + (long)b * j.groups * kChunks * 2;
+    for (int k0 = 0; k0 < CT; k0 += 256) {
+        const int k = k0 + (int)threadIdx.x - sub * across;
+        const bool live = sub < down && k < CT;
+        const float* at = j.x + (long)b * N * CT + (live ? k : 0);
+        double ss = 0.0;
+        constexpr int kAhead = 8;
+        for (int i = n_lo + sub; i < n_hi; i += kAhead * down) {
+            float v[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) {
+                const int node = i + u * down;
+                v[u] = at[(long)(node < n_hi ? node : n_hi - 1) * CT];
+                if (node >= n_hi) v[u] = 0.f;
+            }
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) ss += (double)v[u] * v[u];
+        }
+        __syncthreads();                                           // (the block of positions before this one has been added)
+        sums[threadIdx.x] = live ? ss : 0.0;
+        __syncthreads();
+        const int k_end = k0 + across < CT ? k0 + across : CT;
+        // a wave to a group, the same one in every block: its positions in this block, all rows of a trip
+        for (int g = k0 / per + ((wave - k0 / per) & 3); g * per < k_end; g += 4) {
+            const int lo = g * per > k0 ? g * per : k0, hi = (g + 1) * per < k_end ? (g + 1) * per : k_end;
+            double t = 0.0;
+            for (int q = lo + lane; q < hi; q += kWave)
+                for (int r = 0; r < down; r++) t += sums[r * across + q - k0];
+#pragma unroll
+            for (int d = kWave / 2; d > 0; d >>= 1) t += __shfl_xor(t, d);
+            if (lane == 0) {
+                double* to = partial + ((long)g * kChunks + chunk) * 2;
+                to[1] = lo == g * per ? t : to[1] + t;             // (a group that began in the block before: this lane wrote it there)
+                to[0] = 0.0;
+            }
+        }
+    }
+}
+__global__ void __launch_bounds__(256) tens_apply_kernel(const NormJobs jobs, int N) {
+    int which = 0;
+    while (which + 1 < jobs.count && (int)blockIdx.x >= jobs.job[which + 1].first_block) which++;     // (uniform)
+    const NormJob& j = jobs.job[which];
+    group_apply<0>(j.x, j.chan, nullptr, 0, j.partial, N, j.chan, j.groups, j.T, 0, j.eps, j.gamma, nullptr, nullptr, 0, j.res, j.out,
+                   UpdateVec{}, (int)blockIdx.x - j.first_block);
 }
 
 // Gradient of the tensor norm y = gamma x / s, s = sqrt(eps + mean x^2) over a (box, group):
@@ -399,6 +477,33 @@ int mg_painn_update_post(const float* lrv, int lrv_comp_major, const float* ip, 
     MG_REQUIRE((long)batch * nodes * n == 0 || (lrv && y && ip && out_v), "mg_painn_update_post: null pointer");
     return group_norm(1, ip, n, y + n, 3L * n, batch, nodes, n, groups, 1, eps, gamma, beta, y + 2 * n, 3L * n, res_a, scratch, out_a,
                       1 + lrv_comp_major, UpdateVec{lrv, y, res_v, out_v}, stream);
+}
+
+int mg_tens_group_norms(const mg_tens_norm* norms, int count, int batch, int nodes, void* scratch, mg_stream_t stream) {
+    MG_REQUIRE(count >= 0 && count <= MG_TENS_NORMS && (norms || count == 0), "mg_tens_group_norms: at most %d norms", MG_TENS_NORMS);
+    MG_REQUIRE(batch >= 0 && nodes >= 0 && batch <= 65535, "mg_tens_group_norms: bad sizes, or more than 65535 boxes");
+    NormJobs jobs{};
+    double* partial = static_cast<double*>(scratch);
+    long blocks = 0;
+    for (int k = 0; k < count; k++) {
+        const mg_tens_norm& n = norms[k];
+        MG_REQUIRE(n.chan >= 0 && n.groups > 0 && n.chan % n.groups == 0, "mg_tens_group_norms: bad sizes");
+        MG_REQUIRE(n.comps == 1 || n.comps == 3 || n.comps == 9, "mg_tens_group_norms: comps must be 1, 3 or 9");
+        MG_REQUIRE((long)n.chan * n.comps <= 65536, "mg_tens_group_norms: rows of more than 65536 floats");
+        if ((long)batch * nodes * n.chan == 0) continue;
+        MG_REQUIRE(n.x && n.gamma && n.out && scratch, "mg_tens_group_norms: null pointer");
+        jobs.job[jobs.count++] = NormJob{n.x, n.gamma, n.res, n.out, partial, n.chan, n.groups, n.comps, (int)blocks, n.eps};
+        partial += (size_t)batch * n.groups * kChunks * 2;
+        blocks += ceil_div((long)n.chan * n.comps, 256);
+    }
+    if (jobs.count == 0) return MG_OK;
+    hipStream_t st = (hipStream_t)stream;
+    hipLaunchKernelGGL(tens_stats_kernel, dim3(kChunks, (unsigned)batch, (unsigned)jobs.count), dim3(256), 0, st, jobs, nodes);
+    // (as apply_grid)
+    const long most = ceil_div(4096L * jobs.count, blocks * batch), strips = ceil_div(nodes, 4);
+    hipLaunchKernelGGL(tens_apply_kernel, dim3((unsigned)blocks, (unsigned)(strips < most ? strips : most), (unsigned)batch), dim3(256), 0, st,
+                       jobs, nodes);
+    return check_launch("mg_tens_group_norms");
 }
 
 int mg_tensor_norm_grad_workspace_bytes_of(int batch, int nodes, int chan, int groups, int comps, size_t* bytes) {

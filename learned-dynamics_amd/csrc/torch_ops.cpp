@@ -676,6 +676,39 @@ std::tuple<at::Tensor, at::Tensor> tens_norm_fwd(const at::Tensor& x, const at::
                         scratch.data_ptr(), fp(y), stream_of(x)));
     return {y, scratch};
 }
+// TensGroupNorm.forward of several x (batch, nodes, chan, ..) over the same nodes, with res[k] added: two launches
+Tensors tens_norms(const Tensors& x, const Tensors& gamma, const std::vector<OptTensor>& res, const std::vector<int64_t>& groups,
+                   const std::vector<double>& eps) {
+    const size_t count = x.size();
+    TORCH_CHECK(count >= 1 && count <= MG_TENS_NORMS && gamma.size() == count && res.size() == count && groups.size() == count && eps.size() == count,
+                "tens_norms: up to ", MG_TENS_NORMS, " norms");
+    const int64_t B = x[0].size(0), N = x[0].dim() >= 3 ? x[0].size(1) : -1;
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x[0].device());
+    mg_tens_norm norms[MG_TENS_NORMS];
+    Tensors out;
+    size_t bytes = 0;
+    for (size_t k = 0; k < count; k++) {
+        check_input(x[k], "x");
+        check_input(gamma[k], "gamma");
+        TORCH_CHECK(x[k].dim() >= 3 && x[k].dim() <= 5 && x[k].size(0) == B && x[k].size(1) == N && gamma[k].numel() == x[k].size(2),
+                    "x must have shape (batch, nodes, chan, (3,)^inds)");
+        if (res[k].has_value()) {
+            check_input(*res[k], "res");
+            TORCH_CHECK(res[k]->sizes() == x[k].sizes(), "res has wrong shape");
+        }
+        out.push_back(floats(x[k], x[k].sizes()));
+        int64_t comps = 1;
+        for (int64_t d = 3; d < x[k].dim(); d++) comps *= x[k].size(d);
+        norms[k] = {fp(x[k]), fp(gamma[k]), res[k].has_value() ? fp(*res[k]) : nullptr, fp(out[k]), (int)x[k].size(2), (int)comps,
+                    (int)groups[k], (float)eps[k]};
+        size_t n = 0;
+        check(mg_group_norm_scratch_bytes((int)B, (int)groups[k], &n));
+        bytes += n;
+    }
+    at::Tensor scratch = bytes_like(x[0], std::max<size_t>(bytes, 8));
+    check(mg_tens_group_norms(norms, (int)count, (int)B, (int)N, scratch.data_ptr(), stream_of(x[0])));
+    return out;
+}
 std::tuple<at::Tensor, at::Tensor> tens_norm_bwd(const at::Tensor& dy, const at::Tensor& x, const at::Tensor& gamma, const at::Tensor& scratch,
                                                  int groups, double eps) {
     check_input(dy, "dy");
@@ -1707,6 +1740,7 @@ std::tuple<Tensors, OptTensor, OptTensor> bee_message_bwd(const Tensors& left, c
 void register_ops(pybind11::module_& m) {
     m.def("invalidate_weight_caches", [] { g_epoch.fetch_add(1); });
     m.def("packed_weight", &packed_weight);
+    m.def("tens_norms", &tens_norms);
     m.def("row_absmax", &row_absmax);
     m.def("linear_f16x2", &linear_f16x2);
     m.def("linear_fwd", &linear_fwd);

@@ -2354,6 +2354,13 @@ def group_norm(mode, x, groups, gamma, beta=None, eps=1e-5, mul=None, add=None, 
     return out
 
 
+def tens_group_norms(norms):
+    """group_norm(GN_TENSOR, ..) of up to three (x (batch, nodes, chan, (3,)^inds), groups, gamma, eps, res or None) over the same nodes,
+    x and res contiguous, in the two launches of one."""
+    x, groups, gamma, eps, res = zip(*norms)
+    return _ext.tens_norms(x, gamma, res, groups, eps)
+
+
 # TensGroupNorm.forward with the sums that its adjoint reads, and the adjoint: (x (batch, nodes, chan, ..), gamma, groups, eps) -> (y,
 # sums); (dy, x, gamma, sums, groups, eps) -> (dx, dgamma)
 tens_norm_fwd, tens_norm_bwd = _ext.tens_norm_fwd, _ext.tens_norm_bwd

@@ -672,3 +672,35 @@ def test_displacement_tensors_module(pkg, dims):
     r32 = OL.displacement_tensors(src, 2, 500, r_ref, _to(w, torch.float32), r0, radial_dtype=torch.float64)
     for k, (got, name) in enumerate(zip((A_a, A_v, A_d), "avd")):
         assert_parity(got, r32[k], r64[k], f"DisplacementTensors {dims} A_{name}")
+
+
+@pytest.mark.parametrize("batch,nodes,shapes", [(1, 1, ((8, 0, 8), (16, 1, 8), (8, 2, 4))), (3, 63, ((256, 0, 8), (64, 1, 8), (16, 2, 8))),
+                                                (2, 257, ((300, 0, 5), (96, 1, 3), (64, 2, 1))), (1, 700, ((257, 0, 1), (130, 2, 13)))])
+def test_norms_of_several_tensors_in_the_launches_of_one(ops, batch, nodes, shapes):
+    """tens_group_norms against group_norm tensor by tensor: rows shorter and longer than a workgroup, groups that begin in one block of
+    256 positions and end in another, fewer nodes than chunks.  The sums of squares differ in the order of fp64 additions alone, so
+    the float32 denominators agree, or are neighbours where their rounding is a tie: one unit in the last place of the result."""
+    g = torch.Generator().manual_seed(nodes)
+    jobs = []
+    for k, (chan, rank, groups) in enumerate(shapes):
+        x = torch.randn(batch, nodes, chan, *[3] * rank, generator=g).cuda()
+        jobs.append((x, groups, torch.randn(chan, generator=g).cuda(), 1e-5, torch.randn(x.shape, generator=g).cuda() if k != 1 else None))
+    for y, (x, groups, gamma, eps, res) in zip(ops.tens_group_norms(jobs), jobs):
+        ref = ops.group_norm(ops.GN_TENSOR, x, groups, gamma, None, eps, res=res)
+        assert bool(((y - ref).abs() <= 2.0 ** -23 * (ref.abs() + (res.abs() if res is not None else 0.))).all())
+
+
+def test_norms_with_hooks_are_called_one_by_one(pkg):
+    """SelfTensProds runs its norms in one call only where calling them runs nothing else."""
+    bl = importlib.import_module("learned-dynamics_amd.bee_layers")
+    torch.manual_seed(5)
+    prods, calls = bl.SelfTensProds(32, 16, 8, 64).cuda(), []
+    x = torch.randn(2, 40, 32).cuda(), torch.randn(2, 40, 16, 3).cuda(), torch.randn(2, 40, 8, 3, 3).cuda()
+    with torch.no_grad():
+        together = prods(*x, residual=True)
+        hook = prods.gn_v.register_forward_hook(lambda *a: calls.append(1))
+        apart = prods(*x, residual=True)
+        hook.remove()
+    assert calls == [1]
+    for a, b in zip(together, apart):
+        torch.testing.assert_close(a, b, rtol=1e-6, atol=1e-6)
