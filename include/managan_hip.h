@@ -453,6 +453,11 @@ int mg_mlp_leaky_rowsum_f16x2_workspace_bytes(long rows, int dim, size_t* bytes 
 int mg_mlp_leaky_rowsum_f16x2(const void* packed_W1, const float* b1, const void* packed_W2, const float* b2, const float* x,
                               long rows, int dim_in, int dim, const int* row_ptr, const int* seg, long n_out, void* workspace,
                               float* out, mg_stream_t stream);
+/* The same into rows of out_stride floats (a multiple of 4): a block of columns of a wider matrix.  row_max (n_out, max_stride): its first
+ * dim / 256 entries take the largest magnitude of each 256 columns of the row, bounds for a linear over it.  dim % 256 == 0. */
+int mg_mlp_leaky_rowsum_f16x2_into(const void* packed_W1, const float* b1, const void* packed_W2, const float* b2, const float* x,
+                                   long rows, int dim_in, int dim, const int* row_ptr, const int* seg, long n_out, void* workspace,
+                                   float* out, long out_stride, float* row_max, int max_stride, mg_stream_t stream);
 /* y = act(x W^T + bias) in float64 arithmetic: W (dim_out, dim_in) and bias are the float32 parameters, widened
  * exactly; x (rows, dim_in), every product and sum, the activation and y (rows, dim_out) are double.  The same
  * contraction as nn.Linear inside the reference's MLPs (archs/meanflow_painn8.py:38-51); float64 has no counterpart
@@ -931,6 +936,13 @@ int mg_tensor_linear_f16x2_rowsum_scaled_bound(const void* packed_W, const float
                                                int dim_out, const float* bias, int act, const int* row_ptr,
                                                const int* seg, long n_out, float scale, void* workspace, float* y,
                                                float* out, float bound_mul, float bound_add, mg_stream_t stream);
+/* The same into rows of out_stride floats with their maxima, as mg_mlp_leaky_rowsum_f16x2_into.  base (n_out, dim_out) or NULL:
+ * base[s] += (rows of s) * count_bias, or = with fresh != 0: the bias of a linear applied to the sums. */
+int mg_tensor_linear_f16x2_rowsum_into(const void* packed_W, const float* x, const float* x_rowmax, int x_rowmax_parts,
+                                       long x_rowmax_stride, long rows, int dim_in, int dim_out, const float* bias, int act,
+                                       const int* row_ptr, const int* seg, long n_out, float scale, void* workspace, float* y,
+                                       float* out, long out_stride, float* row_max, int max_stride, const float* count_bias,
+                                       float* base, int fresh, float bound_mul, float bound_add, mg_stream_t stream);
 
 /* The maps lin_l, lin_r, lin_v of Update.forward (archs/meanflow_painn8.py:63-75) and mg_painn_update_pre in one: x_v (rows, n, 3), x_a
  * (rows, n), packed_W the packed weight of the three maps below one another, (3n, n) -> ip, cat and cat_rowmax as there, v (rows, 3, n) =

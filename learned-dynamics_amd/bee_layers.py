@@ -287,6 +287,34 @@ class MLP(nn.Module):
             count = (row_ptr[1:] - row_ptr[:-1]).to(out.dtype)[:, None]
         return out.addcmul_(count, b_last[None, :])
 
+    def takes_linear_summed_over_rows(self, rows, x, add_to=None):
+        """of_linear_summed_over_rows takes x (rows, dim_in of the linear before this MLP) and add_to."""
+        L = self.layers
+        dim, hidden = L[0].in_features, L[0].out_features
+        return (dim % 256 == 0 and ops.rowsum_into_supported(rows, x.shape[1], dim, x)
+                and ops.mlp_rowsum_supported(rows, dim, hidden, x, L[0].bias, L[2].bias, L[4].bias, add_to))
+
+    def of_linear_summed_over_rows(self, W, x, bound, row_ptr, n_out, seg, scale=1.0, add_to=None):
+        """summed_over_rows(psi, plus_identity=True) of psi = x W^T, where it takes_linear_summed_over_rows.  The sums of the hidden rows
+        and of psi are column blocks of one matrix, written there with their row maxima by the kernels that form them, and the first of
+        these adds the counted bias to the result: both node-level linears are one, and no pass measures rows or adds a bias (four
+        launches and two passes over the result less; eight blocks of 256 channels on 2048 nodes 3510 -> 3426 us, on 65 536 nodes
+        67.2 -> 66.3 ms).  The hidden rows come first: the identity's large terms are then added last, and the error against
+        float64 is that of the two linears or less (1.44e-7 against 2.00e-7; the other way round 2.40e-7)."""
+        L = self.layers
+        Wd0, W_last0, b_last0 = self.lin_direct.weight, L[4].weight, L[4].bias
+        tail = _derived(self, ("tail", scale), (Wd0, W_last0), lambda: scale * torch.cat(
+            (W_last0, Wd0 + torch.eye(Wd0.shape[0], device=Wd0.device, dtype=Wd0.dtype)), 1))
+        b_last = b_last0 if scale == 1.0 else _derived(self, ("last_bias_scaled", scale), (b_last0,), lambda: scale * b_last0)
+        dim, hidden = L[0].in_features, L[0].out_features
+        S = torch.empty(n_out, dim + hidden, dtype=torch.float32, device=x.device)
+        maxima = torch.empty(n_out, (dim + hidden) // 256, dtype=torch.float32, device=x.device)
+        out = torch.empty(n_out, dim, dtype=torch.float32, device=x.device) if add_to is None else add_to
+        _, psi = ops.tensor_linear_f16x2_rowsum(W, x, bound, row_ptr, seg, n_out, want_rows=True, into=(S, maxima, hidden),
+                                                count_bias=b_last, base=out, accumulate=add_to is not None)
+        ops.mlp_leaky_rowsum(L[0].weight, L[0].bias, L[2].weight, L[2].bias, psi, row_ptr, seg, n_out, (S, maxima, 0))
+        return ops.tensor_linear_fwd(0, tail, S, out=out, accumulate=True, row_bound=maxima)
+
 
 class DisplacementTensors(nn.Module):
     """archs/diffuser_atoms15.py:206-225: ACE-like embedding of the neighbourhood.  The radial MLP runs per edge
@@ -368,6 +396,9 @@ class Messages(nn.Module):
         bound = emax if ops.get_linear_mode() == ops.LINEAR_F16X2 else None     # row maxima of P0 from the edge kernel
 
         def scalar_channel(bound=bound):
+            add_to = x_a.reshape(rows, -1) if in_place else None
+            if bound is not None and self.mlp_a.takes_linear_summed_over_rows(E, P0, add_to):
+                return self.mlp_a.of_linear_summed_over_rows(Y0, P0, bound, graph.row_ptr, rows, graph.src32, scale=0.1, add_to=add_to)
             if bound is not None and ops.f16x2_rowsum_supported(E, 3 * chan, Y0.shape[0], P0):
                 # psi_a and its sum over the edges of each node from one kernel
                 s_psi, psi_a = ops.tensor_linear_f16x2_rowsum(Y0, P0, bound, graph.row_ptr, graph.src32, rows,
@@ -379,7 +410,7 @@ class Messages(nn.Module):
                 s_psi = None
             return self.mlp_a.summed_over_rows(psi_a, graph.row_ptr, rows, plus_identity=True, bound=bound, scale=0.1,
                                                seg=graph.src32, s_x=s_psi, count=graph.degree,
-                                               add_to=x_a.reshape(rows, -1) if in_place else None)
+                                               add_to=add_to)
         # vector and rank-2 channels: output linears after the edge sum, on node rows (beside the per-edge MLP of the
         # scalar channel when the system is small)
         into_v = dict(out=x_v.reshape(rows, -1, 3), accumulate=True) if in_place else {}

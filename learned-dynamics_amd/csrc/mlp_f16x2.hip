@@ -389,7 +389,7 @@ struct RowsumArgs {
     const float* inv[2];
     const float* bias[2];
     const int* seg;
-    long n_blocks;
+    long n_blocks, out_stride;
     float *slots, *out;
 };
 
@@ -534,7 +534,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 4) mlp_rowsum_f16x2_kernel(con
             if (starts >> (r + 32 * G) & 1) {                      // (never at a row past the end)
                 *to = sum;
                 sum = 0.f;
-                to = a.out + (long)(G ? s_hi : s_lo) * O + col;
+                to = a.out + (long)(G ? s_hi : s_lo) * a.out_stride + col;
             }
         }
         const float v = acc[r >> 2 & 1][0][4 * (r >> 3) + (r & 3)];
@@ -792,15 +792,9 @@ int mg_mlp_leaky_f16x2_adjoint(const mg_mlp_leaky_f16x2_grad* p, mg_stream_t str
 int mg_mlp_leaky_f16x2_residual_forward(const mg_mlp_leaky_f16x2* p, mg_stream_t stream) { return mlp_leaky_forward(p, true, stream); }
 int mg_mlp_leaky_f16x2_residual_adjoint(const mg_mlp_leaky_f16x2_grad* p, mg_stream_t stream) { return mlp_leaky_adjoint(p, true, stream); }
 
-int mg_mlp_leaky_rowsum_f16x2_workspace_bytes(long rows, int dim, size_t* bytes) {
-    MG_REQUIRE(bytes != nullptr && rows >= 0 && dim >= 0, "mg_mlp_leaky_rowsum_f16x2_workspace_bytes: bad argument");
-    *bytes = (size_t)(2 * ceil_div(rows, 32) * dim) * sizeof(float);
-    return MG_OK;
-}
-
-int mg_mlp_leaky_rowsum_f16x2(const void* packed_W1, const float* b1, const void* packed_W2, const float* b2, const float* x,
-                              long rows, int dim_in, int dim, const int* row_ptr, const int* seg, long n_out, void* workspace,
-                              float* out, mg_stream_t stream) {
+static int mlp_rowsum(const void* packed_W1, const float* b1, const void* packed_W2, const float* b2, const float* x, long rows, int dim_in,
+                      int dim, const int* row_ptr, const int* seg, long n_out, void* workspace, float* out, long out_stride, float* row_max,
+                      int max_stride, mg_stream_t stream) {
     MG_REQUIRE(mg_mlp_f16x2_supported(dim_in, dim), "mg_mlp_leaky_rowsum_f16x2: dimensions must be multiples of 32 up to %d", kMaxDim);
     MG_REQUIRE(rows >= 0 && n_out >= 0 && rows < (1L << 31) && n_out < (1L << 31), "mg_mlp_leaky_rowsum_f16x2: bad size");
     if (n_out == 0) return MG_OK;
@@ -815,6 +809,7 @@ int mg_mlp_leaky_rowsum_f16x2(const void* packed_W1, const float* b1, const void
     a.n_blocks = ceil_div(rows, 32);
     a.slots = static_cast<float*>(workspace);
     a.out = out;
+    a.out_stride = out_stride;
     if (rows > 0) {
         const void* packed[2] = {packed_W1, packed_W2};
         const float* bias[2] = {b1, b2};
@@ -832,8 +827,34 @@ int mg_mlp_leaky_rowsum_f16x2(const void* packed_W1, const float* b1, const void
         hipLaunchKernelGGL(mlp_rowsum_f16x2_kernel, dim3((unsigned)ceil_div(rows, 64)), dim3(2 * dim), lds, st, a);
         if (int code = check_launch("mg_mlp_leaky_rowsum_f16x2")) return code;
     }
-    rowsum_finish_kernel<<<dim3((unsigned)ceil_div(n_out * (dim / 4), 256)), dim3(256), 0, st>>>(row_ptr, n_out, a.n_blocks, dim, a.slots, 1.f, out);
+    const dim3 finish((unsigned)ceil_div(n_out * (dim / 4), 256));
+    if (row_max)
+        rowsum_finish_into_kernel<<<finish, dim3(256), 0, st>>>(row_ptr, n_out, a.n_blocks, dim, a.slots, 1.f, out, out_stride, row_max,
+                                                                max_stride, nullptr, nullptr, 0);
+    else
+        rowsum_finish_kernel<<<finish, dim3(256), 0, st>>>(row_ptr, n_out, a.n_blocks, dim, a.slots, 1.f, out);
     return check_launch("rowsum_finish_kernel");
+}
+
+int mg_mlp_leaky_rowsum_f16x2_workspace_bytes(long rows, int dim, size_t* bytes) {
+    MG_REQUIRE(bytes != nullptr && rows >= 0 && dim >= 0, "mg_mlp_leaky_rowsum_f16x2_workspace_bytes: bad argument");
+    *bytes = (size_t)(2 * ceil_div(rows, 32) * dim) * sizeof(float);
+    return MG_OK;
+}
+
+int mg_mlp_leaky_rowsum_f16x2(const void* packed_W1, const float* b1, const void* packed_W2, const float* b2, const float* x,
+                              long rows, int dim_in, int dim, const int* row_ptr, const int* seg, long n_out, void* workspace,
+                              float* out, mg_stream_t stream) {
+    return mlp_rowsum(packed_W1, b1, packed_W2, b2, x, rows, dim_in, dim, row_ptr, seg, n_out, workspace, out, dim, nullptr, 0, stream);
+}
+
+int mg_mlp_leaky_rowsum_f16x2_into(const void* packed_W1, const float* b1, const void* packed_W2, const float* b2, const float* x,
+                                   long rows, int dim_in, int dim, const int* row_ptr, const int* seg, long n_out, void* workspace,
+                                   float* out, long out_stride, float* row_max, int max_stride, mg_stream_t stream) {
+    MG_REQUIRE(row_max && dim % 256 == 0 && out_stride >= dim && out_stride % 4 == 0 && max_stride >= dim / 256,
+               "mg_mlp_leaky_rowsum_f16x2_into: rows of at least dim floats in fours, dim a multiple of 256, and their maxima");
+    return mlp_rowsum(packed_W1, b1, packed_W2, b2, x, rows, dim_in, dim, row_ptr, seg, n_out, workspace, out, out_stride, row_max,
+                      max_stride, stream);
 }
 
 }  // extern "C"

@@ -375,7 +375,7 @@ linear_rowsum_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restr
                            const float* __restrict__ bias, const float* __restrict__ X,
                            const float* __restrict__ xmax, int xmax_parts, long xmax_stride, long R, int I, int O,
                            const int* __restrict__ seg, float* __restrict__ slots, long n_blocks, float scale,
-                           float* __restrict__ Y, float* __restrict__ out, int tiles_n, long tiles_total,
+                           float* __restrict__ Y, float* __restrict__ out, long out_stride, int tiles_n, long tiles_total,
                            float bound_mul, float bound_add) {
     constexpr int kSlice = kFSlice, kRed = kFRed, TN = 32 * NI;
     __shared__ __attribute__((aligned(16))) unsigned char lds[kFLds];
@@ -458,7 +458,7 @@ linear_rowsum_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restr
                 slot_b[col] = sum;
             } else {
                 const long s_id = __shfl(my_seg, r);          // a whole segment inside the block
-                out[s_id * O + col] = scale * sum;
+                out[s_id * out_stride + col] = scale * sum;
             }
         };
         if (nv > 0) {
@@ -741,26 +741,10 @@ int mg_painn_filter_message(const void* packed_W3, const float* bias3, const flo
     return check_launch("painn_message_finish_kernel");
 }
 
-int mg_tensor_linear_f16x2_rowsum_workspace_bytes(long rows, int dim_out, size_t* bytes) {
-    MG_REQUIRE(bytes != nullptr && rows >= 0 && dim_out >= 0, "mg_tensor_linear_f16x2_rowsum_workspace_bytes: bad argument");
-    *bytes = (size_t)(2L * (ceil_div(rows, 32) + 1) * dim_out) * sizeof(float);
-    return MG_OK;
-}
-
-int mg_tensor_linear_f16x2_rowsum(const void* packed_W, const float* x, const float* x_rowmax, int x_rowmax_parts,
-                                  long x_rowmax_stride, long rows, int dim_in, int dim_out, const float* bias, int act,
-                                  const int* row_ptr, const int* seg, long n_out, float scale, void* workspace,
-                                  float* y, float* out, mg_stream_t stream) {
-    return mg_tensor_linear_f16x2_rowsum_scaled_bound(packed_W, x, x_rowmax, x_rowmax_parts, x_rowmax_stride, rows, dim_in,
-                                                      dim_out, bias, act, row_ptr, seg, n_out, scale, workspace, y, out,
-                                                      1.0f, 0.0f, stream);
-}
-
-int mg_tensor_linear_f16x2_rowsum_scaled_bound(const void* packed_W, const float* x, const float* x_rowmax,
-                                               int x_rowmax_parts, long x_rowmax_stride, long rows, int dim_in,
-                                               int dim_out, const float* bias, int act, const int* row_ptr,
-                                               const int* seg, long n_out, float scale, void* workspace, float* y,
-                                               float* out, float bound_mul, float bound_add, mg_stream_t stream) {
+static int linear_rowsum(const void* packed_W, const float* x, const float* x_rowmax, int x_rowmax_parts, long x_rowmax_stride, long rows,
+                         int dim_in, int dim_out, const float* bias, int act, const int* row_ptr, const int* seg, long n_out, float scale,
+                         void* workspace, float* y, float* out, float bound_mul, float bound_add, long out_stride, float* row_max,
+                         int max_stride, const float* count_bias, float* base, int fresh, mg_stream_t stream) {
     MG_REQUIRE(bound_mul >= 0.f && bound_add >= 0.f && bound_mul == bound_mul && bound_add == bound_add,
                "mg_tensor_linear_f16x2_rowsum: the bound's factor and offset must be non-negative numbers");
     MG_REQUIRE(dim_out >= 256 && dim_out % 256 == 0, "mg_tensor_linear_f16x2_rowsum: dim_out must be a multiple of 256 (got %d)", dim_out);
@@ -802,7 +786,7 @@ int mg_tensor_linear_f16x2_rowsum_scaled_bound(const void* packed_W, const float
 #define MG_ROWSUM_TILE(A, S, NI_)                                                                                       \
     linear_rowsum_f16x2_kernel<A, S, NI_><<<dim3((unsigned)grid), dim3(64 * kFW), 0, s>>>(                                \
         planes, w_inv, bias, x, x_rowmax, x_rowmax_parts, x_rowmax_stride, rows, dim_in, dim_out, seg, slots, n_blocks, \
-        scale, y, out, tiles_n, tiles_total, bound_mul, bound_add)
+        scale, y, out, out_stride, tiles_n, tiles_total, bound_mul, bound_add)
         if (y) {
             if (act == 1) MG_ROWSUM_LAUNCH(1, true);
             else if (act == 2) MG_ROWSUM_LAUNCH(2, true);
@@ -816,10 +800,50 @@ int mg_tensor_linear_f16x2_rowsum_scaled_bound(const void* packed_W, const float
 #undef MG_ROWSUM_LAUNCH
         if (int st = check_launch("linear_rowsum_f16x2_kernel")) return st;
     }
-    const long threads = n_out * (dim_out / 4);
-    rowsum_finish_kernel<<<dim3((unsigned)ceil_div(threads, 256)), dim3(256), 0, s>>>(
-        row_ptr, n_out, n_blocks, dim_out, static_cast<const float*>(workspace), scale, out);
+    const dim3 finish((unsigned)ceil_div(n_out * (dim_out / 4), 256));
+    if (row_max)
+        rowsum_finish_into_kernel<<<finish, dim3(256), 0, s>>>(row_ptr, n_out, n_blocks, dim_out, static_cast<const float*>(workspace), scale,
+                                                               out, out_stride, row_max, max_stride, count_bias, base, fresh);
+    else
+        rowsum_finish_kernel<<<finish, dim3(256), 0, s>>>(row_ptr, n_out, n_blocks, dim_out, static_cast<const float*>(workspace), scale, out);
     return check_launch("rowsum_finish_kernel");
+}
+
+int mg_tensor_linear_f16x2_rowsum_workspace_bytes(long rows, int dim_out, size_t* bytes) {
+    MG_REQUIRE(bytes != nullptr && rows >= 0 && dim_out >= 0, "mg_tensor_linear_f16x2_rowsum_workspace_bytes: bad argument");
+    *bytes = (size_t)(2L * (ceil_div(rows, 32) + 1) * dim_out) * sizeof(float);
+    return MG_OK;
+}
+
+int mg_tensor_linear_f16x2_rowsum(const void* packed_W, const float* x, const float* x_rowmax, int x_rowmax_parts,
+                                  long x_rowmax_stride, long rows, int dim_in, int dim_out, const float* bias, int act,
+                                  const int* row_ptr, const int* seg, long n_out, float scale, void* workspace,
+                                  float* y, float* out, mg_stream_t stream) {
+    return mg_tensor_linear_f16x2_rowsum_scaled_bound(packed_W, x, x_rowmax, x_rowmax_parts, x_rowmax_stride, rows, dim_in,
+                                                      dim_out, bias, act, row_ptr, seg, n_out, scale, workspace, y, out,
+                                                      1.0f, 0.0f, stream);
+}
+
+int mg_tensor_linear_f16x2_rowsum_scaled_bound(const void* packed_W, const float* x, const float* x_rowmax,
+                                               int x_rowmax_parts, long x_rowmax_stride, long rows, int dim_in,
+                                               int dim_out, const float* bias, int act, const int* row_ptr,
+                                               const int* seg, long n_out, float scale, void* workspace, float* y,
+                                               float* out, float bound_mul, float bound_add, mg_stream_t stream) {
+    return linear_rowsum(packed_W, x, x_rowmax, x_rowmax_parts, x_rowmax_stride, rows, dim_in, dim_out, bias, act, row_ptr, seg, n_out,
+                         scale, workspace, y, out, bound_mul, bound_add, dim_out, nullptr, 0, nullptr, nullptr, 0, stream);
+}
+
+int mg_tensor_linear_f16x2_rowsum_into(const void* packed_W, const float* x, const float* x_rowmax, int x_rowmax_parts, long x_rowmax_stride,
+                                       long rows, int dim_in, int dim_out, const float* bias, int act, const int* row_ptr, const int* seg,
+                                       long n_out, float scale, void* workspace, float* y, float* out, long out_stride, float* row_max,
+                                       int max_stride, const float* count_bias, float* base, int fresh, float bound_mul, float bound_add,
+                                       mg_stream_t stream) {
+    MG_REQUIRE(row_max && out_stride >= dim_out && out_stride % 4 == 0 && max_stride >= dim_out / 256,
+               "mg_tensor_linear_f16x2_rowsum_into: rows of at least dim_out floats in fours, and their maxima");
+    MG_REQUIRE(!base || (count_bias && aligned16(base) && aligned16(count_bias)),
+               "mg_tensor_linear_f16x2_rowsum_into: the base takes a bias, both 16-byte aligned");
+    return linear_rowsum(packed_W, x, x_rowmax, x_rowmax_parts, x_rowmax_stride, rows, dim_in, dim_out, bias, act, row_ptr, seg, n_out,
+                         scale, workspace, y, out, bound_mul, bound_add, out_stride, row_max, max_stride, count_bias, base, fresh, stream);
 }
 
 int mg_painn_filter_hidden(const float* r_ij, long n_edges, float rmax, const float* W1, long w1_stride_o,

@@ -1965,11 +1965,15 @@ def f16x2_rowsum_supported(rows, dim_in, dim_out, x):
             and rows >= 4096 and x.data_ptr() % 16 == 0)
 
 
-def tensor_linear_f16x2_rowsum(W, x, x_bound, row_ptr, seg, n_out, bias=None, act=ACT_NONE, scale=1.0, want_rows=False):
+def tensor_linear_f16x2_rowsum(W, x, x_bound, row_ptr, seg, n_out, bias=None, act=ACT_NONE, scale=1.0, want_rows=False, into=None,
+                               count_bias=None, base=None, accumulate=False):
     """(out, y): out[s] = scale * sum over the rows r of segment s of act(bias + W x[r]) (n_out, dim_out); y is the
     per-row result (rows, dim_out) when want_rows is set, else None.  Rows are sorted by segment: seg (rows,) int32
     ascending, row_ptr its CSR form.  x_bound: (rows, parts) or (1, parts) upper bounds of the row maxima of |x|, or
-    a ScaledBound of such an array."""
+    a ScaledBound of such an array.
+    into = (S, maxima, col), sizes where rowsum_into_supported: the sums go to columns col .. of S (n_out, wider) and the largest
+    magnitude of each 256 columns to maxima (n_out, S.size(1) / 256); out is then that block of S.  base (n_out, dim_out) then takes the
+    rows of each segment times count_bias, on top of what it holds with accumulate: a bias after the sum."""
     bound_mul, bound_add = 1.0, 0.0
     if isinstance(x_bound, ScaledBound):
         x_bound, bound_mul, bound_add = x_bound.base, x_bound.mul, x_bound.add
@@ -1989,6 +1993,8 @@ def tensor_linear_f16x2_rowsum(W, x, x_bound, row_ptr, seg, n_out, bias=None, ac
         if bias.numel() != dim_out:
             raise RuntimeError("bias must have dim_out elements")
     dev = x.device
+    if into is not None and not rowsum_into_supported(rows, dim_in, dim_out, x):
+        raise RuntimeError("into takes the sizes of rowsum_into_supported")
     if rows and dim_out % 256 == 0 and _lib.mg_tensor_linear_f16x2_splits_k(rows, dim_in, dim_out):
         # few rows: 256-row tiles would leave most of the chip idle
         y = tensor_linear_f16x2(W, x, ScaledBound(x_bound, bound_mul, bound_add), bias=bias, act=act)
@@ -1997,10 +2003,23 @@ def tensor_linear_f16x2_rowsum(W, x, x_bound, row_ptr, seg, n_out, bias=None, ac
     nbytes = ctypes.c_size_t(0)
     L.check(_lib.mg_tensor_linear_f16x2_rowsum_workspace_bytes(rows, dim_out, ctypes.byref(nbytes)))
     with _on(dev):
-        out = torch.empty(n_out, dim_out, dtype=torch.float32, device=dev)
+        out = _rowsum_block(into, n_out, dim_out) if into is not None else torch.empty(n_out, dim_out, dtype=torch.float32, device=dev)
         y = torch.empty(rows, dim_out, dtype=torch.float32, device=dev) if want_rows else None
         work = torch.empty(nbytes.value // 4, dtype=torch.float32, device=dev)
         stride = 0 if x_bound.size(0) == 1 else int(x_bound.size(1))
+        if into is not None:
+            if base is not None:
+                _check_input(base, "base")
+                _check_input(count_bias, "count_bias")
+                if tuple(base.shape) != (n_out, dim_out) or count_bias.numel() != dim_out:
+                    raise RuntimeError("base must be (n_out, dim_out) and count_bias dim_out elements")
+            maxima = into[1]
+            L.check(_lib.mg_tensor_linear_f16x2_rowsum_into(
+                _p(packed_weight_f16x2(W)), _p(x), _p(x_bound), int(x_bound.size(1)), stride, rows, dim_in, dim_out,
+                _p(bias), int(act), _p(row_ptr), _p(seg), int(n_out), float(scale), _p(work), _p(y), _p(out), out.stride(0),
+                _p(maxima[:, into[2] // 256:]), maxima.size(1), _p(count_bias), _p(base), int(not accumulate), bound_mul, bound_add,
+                _stream()))
+            return out, y
         L.check(_lib.mg_tensor_linear_f16x2_rowsum_scaled_bound(
             _p(packed_weight_f16x2(W)), _p(x), _p(x_bound), int(x_bound.size(1)), stride, rows, dim_in, dim_out,
             _p(bias), int(act), _p(row_ptr), _p(seg), int(n_out), float(scale), _p(work), _p(y), _p(out),
@@ -2017,9 +2036,26 @@ def mlp_rowsum_supported(rows, dim_in, dim, x, *biases):
             and bool(_lib.mg_mlp_f16x2_supported(int(dim_in), int(dim))))
 
 
-def mlp_leaky_rowsum(W1, b1, W2, b2, x, row_ptr, seg, n_out):
+def rowsum_into_supported(rows, dim_in, dim_out, x):
+    """tensor_linear_f16x2_rowsum writes the sums as a block of a wider matrix: where it runs as one kernel."""
+    return (f16x2_rowsum_supported(rows, dim_in, dim_out, x)
+            and not _lib.mg_tensor_linear_f16x2_splits_k(int(rows), int(dim_in), int(dim_out)))
+
+
+def _rowsum_block(into, n_out, dim):
+    S, maxima, col = into
+    _check_input(S, "S")
+    _check_input(maxima, "maxima")
+    if (S.dim() != 2 or S.size(0) != n_out or S.size(1) % 256 or col % 256 or dim % 256 or not 0 <= col <= S.size(1) - dim
+            or tuple(maxima.shape) != (n_out, S.size(1) // 256)):
+        raise RuntimeError("into must be (n_out, wider) sums, their maxima and a first column, in multiples of 256 columns")
+    return S[:, col:col + dim]
+
+
+def mlp_leaky_rowsum(W1, b1, W2, b2, x, row_ptr, seg, n_out, into=None):
     """out[s] = sum over the rows r of segment s of f(W2 f(W1 x[r] + b1) + b2) with f = LeakyReLU(0.1): (n_out, dim).  Rows are
-    sorted by segment: seg (rows,) int32 ascending, row_ptr its CSR form.  The hidden rows are never stored."""
+    sorted by segment: seg (rows,) int32 ascending, row_ptr its CSR form.  The hidden rows are never stored.
+    into: as for tensor_linear_f16x2_rowsum (dim a multiple of 256)."""
     for t, nm in ((W1, "W1"), (W2, "W2"), (x, "x"), (b1, "b1"), (b2, "b2")):
         if t is not None or nm in ("W1", "W2", "x"):
             _check_input(t, nm)
@@ -2035,8 +2071,13 @@ def mlp_leaky_rowsum(W1, b1, W2, b2, x, row_ptr, seg, n_out):
     nbytes = ctypes.c_size_t(0)
     L.check(_lib.mg_mlp_leaky_rowsum_f16x2_workspace_bytes(rows, dim, ctypes.byref(nbytes)))
     with _on(x.device):
-        out = torch.empty(n_out, dim, dtype=torch.float32, device=x.device)
+        out = _rowsum_block(into, n_out, dim) if into is not None else torch.empty(n_out, dim, dtype=torch.float32, device=x.device)
         work = torch.empty(nbytes.value // 4, dtype=torch.float32, device=x.device)
+        if into is not None:
+            L.check(_lib.mg_mlp_leaky_rowsum_f16x2_into(
+                _p(packed_weight_f16x2(W1)), _p(b1), _p(packed_weight_f16x2(W2)), _p(b2), _p(x), rows, dim_in, dim, _p(row_ptr), _p(seg),
+                int(n_out), _p(work), _p(out), out.stride(0), _p(into[1][:, into[2] // 256:]), into[1].size(1), _stream()))
+            return out
         L.check(_lib.mg_mlp_leaky_rowsum_f16x2(_p(packed_weight_f16x2(W1)), _p(b1), _p(packed_weight_f16x2(W2)), _p(b2), _p(x),
                                                rows, dim_in, dim, _p(row_ptr), _p(seg), int(n_out), _p(work), _p(out), _stream()))
     return out

@@ -232,6 +232,48 @@ def _summed(pkg, dim, rows, bias_offset=0):
     return error(got), error(reference(torch.float32))
 
 
+@pytest.mark.parametrize("rows, dim_in, in_place", [(6177, 96, True), (7001, 64, False)])
+def test_linear_and_mlp_summed_over_segments_as_one_matrix(bee, ops, rows, dim_in, in_place):
+    """The sums of a linear's rows and of the MLP's hidden rows as blocks of one matrix, against the same sums apart: the hidden rows'
+    sums to the bit, their maxima exact, the result as close to float64 (rounding of 768 products and of the additions to the base, with
+    empty segments and segments of one row to hundreds)."""
+    torch.manual_seed(rows)
+    mlp = bee.MLP(256).cuda()
+    g = torch.Generator().manual_seed(rows)
+    W = (torch.randn(256, dim_in, generator=g) * dim_in ** -0.5).cuda()
+    x = torch.randn(rows, dim_in, generator=g).cuda()
+    row_ptr, seg = (t.int().cuda() for t in _segments(rows, 7))
+    n_out = row_ptr.numel() - 1
+    base = torch.randn(n_out, 256, generator=g).cuda() if in_place else None
+    with torch.no_grad():
+        mlp.layers[4].bias.normal_()
+        bound = ops.row_absmax(x)
+        assert mlp.takes_linear_summed_over_rows(rows, x, base)
+        out = mlp.of_linear_summed_over_rows(W, x, bound, row_ptr, n_out, seg, 0.1, base.clone() if in_place else None)
+        s_psi, psi = ops.tensor_linear_f16x2_rowsum(W, x, bound, row_ptr, seg, n_out, want_rows=True)
+        apart = mlp.summed_over_rows(psi, row_ptr, n_out, plus_identity=True, seg=seg, s_x=s_psi, scale=0.1,
+                                     add_to=base.clone() if in_place else None)
+        L = mlp.layers
+        s_h = ops.mlp_leaky_rowsum(L[0].weight, L[0].bias, L[2].weight, L[2].bias, psi, row_ptr, seg, n_out)
+        S, maxima = torch.full((n_out, 1024), 7., device="cuda"), torch.full((n_out, 4), 7., device="cuda")
+        count = torch.empty(n_out, 256, device="cuda")
+        ops.tensor_linear_f16x2_rowsum(W, x, bound, row_ptr, seg, n_out, into=(S, maxima, 0), count_bias=L[4].bias, base=count)
+        ops.mlp_leaky_rowsum(L[0].weight, L[0].bias, L[2].weight, L[2].bias, psi, row_ptr, seg, n_out, (S, maxima, 256))
+    assert torch.equal(S[:, :256], s_psi) and torch.equal(S[:, 256:768], s_h) and bool((S[:, 768:] == 7).all())
+    assert torch.equal(maxima, S.view(n_out, 4, 256).abs().amax(2))
+    n = (row_ptr[1:] - row_ptr[:-1]).double()[:, None]
+    assert torch.equal(count, (n * L[4].bias.double()).float())
+    w = lambda t: t.detach().double()
+    ref = 0.1 * (s_psi.double() @ w(mlp.lin_direct.weight).t() + s_psi.double() + s_h.double() @ w(L[4].weight).t() + n * w(L[4].bias))
+    ref = ref + base.double() if in_place else ref
+    error = lambda y: float((y.double() - ref).norm() / ref.norm())
+    assert error(out) <= 3e-7 and error(out) <= 1.2 * error(apart)
+    # an unaligned base keeps the general path; sizes and columns that do not fit are refused
+    assert not mlp.takes_linear_summed_over_rows(rows, x, torch.zeros(n_out * 256 + 1, device="cuda")[1:].view(n_out, 256))
+    with pytest.raises(RuntimeError):
+        ops.tensor_linear_f16x2_rowsum(W, x, bound, row_ptr, seg, n_out, into=(S, maxima, 800))
+
+
 def test_narrow_layers_summed_over_segments_stay_in_fp32(bee, ops, monkeypatch):
     """A linear of 32 columns has fp32 arithmetic: the kernel of 22-bit pieces takes a layer from 64 columns on."""
     x = torch.zeros(5000, 64).cuda()
