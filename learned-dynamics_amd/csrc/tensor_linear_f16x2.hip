@@ -544,7 +544,14 @@ linear_rows_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restric
 // 32 rows x 32 NI columns and its WAVES waves split K: wave w takes chunks w, w + WAVES, ... with private
 // accumulators, reads its W fragments straight from the packed planes (L2 resident; no LDS, no barrier in the loop),
 // and the partial tiles are summed through LDS in wave order, so the result does not depend on timing.
-template <int WAVES, int NI>
+// With a workgroup to a CU the reductions of several chunks a wave (ONE false) are bound by the chain bound of the row -> first chunk ->
+// .. -> old value of y, and by the cache's lookups: the bounds (four parts at once) and the first chunk are requested together, the old
+// values before the barrier, and a chunk of x is read eight lanes to a row, 128 bytes at a time, and handed to the lanes that multiply it
+// through this wave's own part of LDS (a lane to a row, 16 bytes at a time, asks for 32 lines with every load, four times over).  6144 rows
+// x 1280 -> 64 onto y 17.0 -> 14.3 us, 900 rows 12.1 -> 10.1; 9216 x 1280 -> 16 19.5 -> 16.2; 2048 x 768 -> 256 onto y 12.9 -> 11.4;
+// 512 -> 512 at 337 rows 8.1 -> 7.6, at 3072 19.4 -> 18.0.  A wave with one chunk at most (ONE) has nothing to gain from either and keeps
+// the straight order (2048 x 256 -> 256 8.0 against 8.3 us, 6144 x 64 -> 256 9.2 against 9.8).
+template <int WAVES, int NI, bool ONE>
 __global__ void __launch_bounds__(64 * WAVES)
 linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __restrict__ w_inv,
                                 const float* __restrict__ X, long x_stride, const float* __restrict__ xmax,
@@ -555,33 +562,36 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
                                 long bias_rows) {
     constexpr int TN = 32 * NI, THREADS = 64 * WAVES;
     constexpr int kPitch = TN + 1;                            // floats per row of a partial tile
-    __shared__ float partial[WAVES][32 * kPitch];
+    constexpr int kTile = 32 * kPitch > 1024 ? 32 * kPitch : 1024;
+    __shared__ __attribute__((aligned(16))) float partial[WAVES][kTile];
     __shared__ float inv_sx[32], wave_max[WAVES][32];
 
-    const long tile_m = blockIdx.x / tiles_n;
+    // (choose_splitk: at most 49 152 rows, R O in 21 bits)
+    const unsigned tile_m = blockIdx.x / (unsigned)tiles_n;
     const int tile_n = (int)(blockIdx.x - tile_m * tiles_n);
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int m = lane & 31, g = lane >> 5;
-    const long r0 = tile_m * 32;
+    const unsigned r0 = tile_m * 32;
     const int n0 = tile_n * TN;
     const long plane_elems = (long)O_pad * I;
 
-    const long my_row = r0 + m;
-    const long ld_row = my_row < R ? my_row : R - 1;
-    const float* xrow = X + ld_row * x_stride + 16 * g;
+    const unsigned my_row = r0 + m, n_rows = (unsigned)R;
+    const unsigned ld_row = my_row < n_rows ? my_row : n_rows - 1;
+    // Piece q (16 bytes) of a chunk's row r lies at q ^ (r / 2) % 8: 16 lanes read 16 different places of the 256 bytes that LDS delivers at once.
+    float* const stage = partial[wave];
+    unsigned piece_row[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const unsigned r = r0 + 8 * j + lane / 8;
+        piece_row[j] = r < n_rows ? r : n_rows - 1;
+    }
     float sx;
     auto set_scale = [&](float amax) {
         float inv;
         sx = pow2_scale(amax, &inv);
         if (wave == 0 && g == 0) inv_sx[m] = beyond_split(amax) ? __builtin_nanf("") : inv;
     };
-    if (xmax) {                                               // (uniform)
-        float amax = 0.f;
-        const float* xm = xmax + (ld_row / xmax_div) * xmax_stride;
-        for (int p = 0; p < xmax_parts; p++) amax = fmaxf(amax, xm[p]);
-        set_scale(fmaf(amax, bound_mul, bound_add));
-    }
     // lane's fragment of W for MFMA step s, column block ni: row n0 + 32 ni + m, k = k0 + 16 g + 8 s .. + 8
     const _Float16* wrow = Wp + packed_piece(n0, lane, I);
 
@@ -595,6 +605,12 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
         float4 a[4];
         halfx8 wh[NI][2], wl[NI][2];
     };
+    auto load_pieces = [&](float4 (&a)[4], int k0) {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            a[j] = ONE ? *reinterpret_cast<const float4*>(X + (long)ld_row * x_stride + k0 + 16 * g + 4 * j)
+                       : *reinterpret_cast<const float4*>(X + (long)piece_row[j] * x_stride + k0 + 4 * (lane & 7));
+    };
     auto load = [&](Chunk& c, int k0) {
 #pragma unroll
         for (int ni = 0; ni < NI; ni++)
@@ -603,8 +619,18 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
                 c.wh[ni][s2] = *reinterpret_cast<const halfx8*>(wrow + (long)ni * 32 * I + 32L * k0 + 512 * s2);
                 c.wl[ni][s2] = *reinterpret_cast<const halfx8*>(wrow + plane_elems + (long)ni * 32 * I + 32L * k0 + 512 * s2);
             }
+        load_pieces(c.a, k0);
+    };
+    auto hand_over = [&](Chunk& c) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) c.a[j] = *reinterpret_cast<const float4*>(xrow + k0 + 4 * j);
+        for (int j = 0; j < 4; j++) {
+            const int r = 8 * j + lane / 8;
+            *reinterpret_cast<float4*>(stage + 32 * r + 4 * ((lane & 7) ^ (r / 2 & 7))) = c.a[j];
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < 4; j++) c.a[j] = *reinterpret_cast<const float4*>(stage + 32 * m + 4 * ((4 * g + j) ^ (m / 2 & 7)));
+        __builtin_amdgcn_wave_barrier();
     };
     auto compute = [&](const Chunk& c) {
 #pragma unroll
@@ -624,38 +650,93 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
             }
         }
     };
-    // this wave's chunks, the next one requested before the current one is consumed
     const int chunks = I / kCK;
     Chunk cur, nxt;
-    if (wave < chunks) load(cur, wave * kCK);
+    const float* const xm = xmax ? xmax + (long)(ld_row / (unsigned)xmax_div) * xmax_stride : nullptr;
+    if constexpr (ONE) {
+        if (xmax) {                                           // (uniform)
+            float amax = 0.f;
+            for (int p = 0; p < xmax_parts; p++) amax = fmaxf(amax, xm[p]);
+            set_scale(fmaf(amax, bound_mul, bound_add));
+        }
+        if (wave < chunks) load(cur, wave * kCK);
+    } else {
+        float part[4] = {0.f, 0.f, 0.f, 0.f};
+        if (xmax) {
+#pragma unroll
+            for (int p = 0; p < 4; p++) part[p] = xm[p < xmax_parts ? p : 0];
+        }
+        if (wave < chunks) load(cur, wave * kCK);
+        if (xmax) {
+            float amax = fmaxf(fmaxf(fmaxf(0.f, part[0]), fmaxf(part[1], part[2])), part[3]);
+            for (int p = 4; p < xmax_parts; p++) amax = fmaxf(amax, xm[p]);
+            set_scale(fmaf(amax, bound_mul, bound_add));
+        }
+    }
     if (!xmax) {                                              // the rows' own maxima, as row_absmax_kernel takes them
-        float amax = 0.f;
+        float mx[4] = {0.f, 0.f, 0.f, 0.f};
         auto largest = [&](const float4 (&a)[4]) {
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                amax = fmaxf(fmaxf(amax, fmaxf(fabsf(a[j].x), fabsf(a[j].y))), fmaxf(fabsf(a[j].z), fabsf(a[j].w)));
+            for (int j = 0; j < 4; j++) mx[j] = fmaxf(fmaxf(mx[j], fmaxf(fabsf(a[j].x), fabsf(a[j].y))), fmaxf(fabsf(a[j].z), fabsf(a[j].w)));
         };
         if (wave < chunks) largest(cur.a);
         for (int c = wave + WAVES; c < chunks; c += WAVES) {
             float4 a[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) a[j] = *reinterpret_cast<const float4*>(xrow + c * kCK + 4 * j);
+            load_pieces(a, c * kCK);
             largest(a);
         }
-        amax = fmaxf(amax, __shfl_xor(amax, 32));
-        if (g == 0) wave_max[wave][m] = amax;
+        if constexpr (ONE) {
+            mx[0] = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]));
+            mx[0] = fmaxf(mx[0], __shfl_xor(mx[0], 32));
+            if (g == 0) wave_max[wave][m] = mx[0];
+        } else
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+#pragma unroll
+            for (int d = 1; d < 8; d <<= 1) mx[j] = fmaxf(mx[j], __shfl_xor(mx[j], d));
+            if ((lane & 7) == 0) wave_max[wave][8 * j + lane / 8] = mx[j];
+        }
         __syncthreads();
+        float amax = 0.f;
 #pragma unroll
         for (int w = 0; w < WAVES; w++) amax = fmaxf(amax, wave_max[w][m]);
-        if (tile_n == 0 && wave == 0 && g == 0 && my_row < R) xmax_out[my_row] = amax;
+        if (tile_n == 0 && wave == 0 && g == 0 && my_row < n_rows) xmax_out[my_row] = amax;
         set_scale(amax);
     }
+    if constexpr (ONE) {
+        if (wave < chunks) compute(cur);
+    } else
     for (int c = wave; c < chunks; c += WAVES) {
         const bool more = c + WAVES < chunks;
         if (more) load(nxt, (c + WAVES) * kCK);
+        hand_over(cur);
         compute(cur);
         if (more) cur = nxt;
     }
+    // a thread finishes the elements e = tid, tid + THREADS, ...: row e / TN, column e % TN (the lanes of a row are neighbours, so its
+    // maximum is a shuffle away)
+    constexpr int kPer = 32 * TN / THREADS;
+    static_assert(32 * TN % THREADS == 0 && THREADS % TN == 0 && TN <= 64, "whole rows per pass, a row within a wave");
+    const int my_n = n0 + tid % TN;
+    float iw = 0.f, my_bias = 0.f, was[kPer];
+    unsigned at[kPer];
+    auto request = [&] {
+        if (my_n < O) {
+            iw = w_inv[my_n];
+            my_bias = bias ? bias[my_n] : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < kPer; j++) {
+            const unsigned r = r0 + (tid + THREADS * j) / TN;
+            at[j] = r * O + my_n;
+            if (out_T != 1) {                                 // (uniform)
+                const unsigned row = r / (unsigned)out_T;
+                at[j] = (row * O + my_n) * out_T + (r - row * out_T);
+            }
+            was[j] = accumulate && r < n_rows && my_n < O ? Y[at[j]] : 0.f;
+        }
+    };
+    if (!ONE) request();
     // partial tiles -> LDS; accumulator register q of block ni is row 8 (q / 4) + 4 g + q % 4, column 32 ni + m
 #pragma unroll
     for (int ni = 0; ni < NI; ni++)
@@ -663,10 +744,7 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
         for (int q = 0; q < 16; q++)
             partial[wave][(8 * (q / 4) + 4 * g + (q % 4)) * kPitch + 32 * ni + m] = acc[ni][q];
     __syncthreads();
-    // a thread finishes the elements e = tid, tid + THREADS, ...: row e / TN, column e % TN (the TN / 1 lanes of a
-    // row are neighbours, so its maximum is a shuffle away)
-    constexpr int kPer = 32 * TN / THREADS;
-    static_assert(32 * TN % THREADS == 0 && THREADS % TN == 0 && TN <= 64, "whole rows per pass, a row within a wave");
+    if (ONE) request();
     bool odd = false;                                         // an element of a row or column that the pieces cannot carry
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
@@ -675,20 +753,14 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
         float sum = 0.f;
 #pragma unroll
         for (int w = 0; w < WAVES; w++) sum += partial[w][rl * kPitch + col];
-        const long r = r0 + rl;
-        const int n = n0 + col;
+        const unsigned r = r0 + rl;
         float v = 0.f;
-        if (r < R && n < O) {
-            const float isx = inv_sx[rl], iw = w_inv[n], bv = bias && r < bias_rows ? bias[n] : 0.f;
-            long addr = r * O + n;
-            if (out_T != 1) {                                 // (uniform)
-                const long row = r / out_T;
-                addr = (row * O + n) * out_T + (r - row * out_T);
-            }
+        if (r < n_rows && my_n < O) {
+            const float isx = inv_sx[rl];
             if (isx == isx && iw == iw) {
-                v = activate(sum * isx * iw + bv, act);
-                if (accumulate) v += Y[addr];
-                Y[addr] = v;
+                v = activate(sum * isx * iw + ((long)r < bias_rows ? my_bias : 0.f), act);
+                if (accumulate) v += was[j];
+                Y[at[j]] = v;
             } else {
                 odd = true;
                 v = __builtin_inff();                         // (no bound: the next layer takes the row in fp32)
@@ -698,19 +770,19 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
             float mx = fabsf(v);
 #pragma unroll
             for (int d = 1; d < TN; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
-            if (col == 0 && r < R) ymax[r * tiles_n + tile_n] = mx;
+            if (col == 0 && r < n_rows) ymax[r * tiles_n + tile_n] = mx;
         }
     }
     if (odd) {
 #pragma unroll 1
         for (int j = 0; j < kPer; j++) {
-            const int e = tid + THREADS * j, rl = e / TN, n = n0 + e - rl * TN;
-            const long r = r0 + rl;
-            if (r >= R || n >= O) continue;
-            const float isx = inv_sx[rl], iw = w_inv[n];
+            const int rl = (tid + THREADS * j) / TN;
+            const unsigned r = r0 + rl;
+            if (r >= n_rows || my_n >= O) continue;
+            const float isx = inv_sx[rl];
             if (isx == isx && iw == iw) continue;
-            const long row = r / out_T, addr = (row * O + n) * out_T + (r - row * out_T);
-            const float v = activate(row_in_fp32(X + r * x_stride, Wp, plane_elems, n, I, iw) + (bias && r < bias_rows ? bias[n] : 0.f), act);
+            const unsigned row = r / (unsigned)out_T, addr = (row * O + my_n) * out_T + (r - row * out_T);
+            const float v = activate(row_in_fp32(X + (long)r * x_stride, Wp, plane_elems, my_n, I, iw) + ((long)r < bias_rows ? my_bias : 0.f), act);
             Y[addr] = accumulate ? v + Y[addr] : v;
         }
     }
@@ -957,8 +1029,10 @@ static int run_strided(const mg_f16x2_linear* args, long x_stride, float* x_rowm
         MG_REQUIRE(tiles <= 0x7fffffffL, "mg_tensor_linear_f16x2: grid too large (rows=%ld)", a.rows);
 #define MG_SPLITK(WV, N)                                                                                                   \
     if (sk.waves == WV && sk.ni == N)                                                                                      \
-        hipLaunchKernelGGL((linear_rows_splitk_f16x2_kernel<WV, N>), dim3((unsigned)tiles), dim3(64 * WV), 0, st, planes,  \
-                           w_inv, a.x, x_stride, given, x_rowmax_out, a.x_rowmax_parts, a.x_rowmax_stride, a.x_rows_per_bound, \
+        hipLaunchKernelGGL((a.dim_in <= kCK * WV ? linear_rows_splitk_f16x2_kernel<WV, N, true>                            \
+                                                 : linear_rows_splitk_f16x2_kernel<WV, N, false>),                         \
+                           dim3((unsigned)tiles), dim3(64 * WV), 0, st, planes, w_inv, a.x, x_stride, given, x_rowmax_out,  \
+                           a.x_rowmax_parts, a.x_rowmax_stride, a.x_rows_per_bound < 0x7fffffffL ? a.x_rows_per_bound : 0x7fffffffL, \
                            a.rows, a.dim_in, a.dim_out, O_pad, a.bias, a.act, a.accumulate, a.y, a.y_rowmax, tiles_n, a.out_comps, \
                            a.bound_mul, a.bound_add, a.bias_rows)
         MG_SPLITK(8, 1);

@@ -948,3 +948,36 @@ def test_few_inputs_of_rank_two_by_component_and_by_channel(rows, dim_in, dim_ou
         assert torch.equal(ops.tensor_linear_fwd(2, W, x, out=base.clone(), accumulate=True, y_layout=ops.LAYOUT_COMP_CHAN), y + base)
         ref = torch.einsum("oi,nixy->noxy", W.double().cpu(), x.double().cpu()).reshape(rows, dim_out, 9)
         torch.testing.assert_close(by_channel.cpu().double().reshape(rows, dim_out, 9), ref, rtol=1e-5, atol=1e-6 * dim_in)
+
+
+@pytest.mark.parametrize("rows, dim_in, dim_out, comps", [
+    (1, 288, 64, 1), (33, 256, 256, 1), (95, 544, 40, 1), (31, 1280, 16, 1), (333, 1280, 64, 3), (2050, 160, 70, 1), (1800, 320, 96, 9)])
+def test_reductions_split_over_waves_with_one_chunk_and_several(ops, rows, dim_in, dim_out, comps):
+    """Onto values that are there, row bounds in one part, four and seven (the bound is their maximum: the same bits), rows and columns
+    that end inside a tile, components.  22-bit pieces and fp32 sums: 2^-21 of the norms of the rows that are multiplied."""
+    g = torch.Generator().manual_seed(rows)
+    W = torch.randn(dim_out, dim_in, generator=g).cuda()
+    x = (torch.randn(rows, dim_in, generator=g) * torch.exp(torch.randn(rows, 1, generator=g))).cuda()
+    nodes = -(-rows // comps)
+    x = torch.cat([x, x[:nodes * comps - rows]])
+    base = torch.randn((nodes, dim_out, comps) if comps > 1 else (nodes, dim_out), generator=g).cuda()
+    bound = ops.row_absmax(x)
+    low = torch.zeros_like(bound)
+
+    def onto(b):
+        return ops.tensor_linear_f16x2(W, x, b, out=base.clone(), accumulate=True, out_comps=comps)
+    y = onto(bound)
+    ref = (x.double() @ W.double().t()).view(nodes, comps, dim_out).transpose(1, 2).reshape(base.shape) + base.double()
+    size = (x.double().norm(dim=1)[:, None] * W.double().norm(dim=1)).view(nodes, comps, dim_out).transpose(1, 2).reshape(base.shape)
+    assert float(((y.double() - ref).abs() / (size + base.abs())).max()) <= 2.0 ** -21
+    for parts in ([low, low, bound, low], [low, low, low, low, low, low, bound], [low, low, low, low, bound]):
+        assert torch.equal(onto(torch.cat(parts, 1)), y)
+    # a row without a bound that the pieces can carry, in every tile but its own the same bits
+    x[rows // 2, 1] = 2.0 ** 100
+    z = onto(ops.row_absmax(x))
+    ref = (x.double() @ W.double().t()).view(nodes, comps, dim_out)[rows // 2 // comps, rows // 2 % comps]
+    pick = lambda t: t.view(nodes, dim_out, comps)[rows // 2 // comps, :, rows // 2 % comps]
+    assert float(((pick(z).double() - ref) / ref).abs().max()) <= 1e-6
+    keep = torch.ones(nodes, dtype=torch.bool, device="cuda")
+    keep[rows // 2 // comps] = False
+    assert torch.equal(z[keep], y[keep])
