@@ -388,24 +388,30 @@ int launch_rows(const float* W, long so, long si, const float* X, long R, int I,
 
 
 // Several linears whose operands lie side by side in rows of x, summed: y = sum_p x[:, p C .. + C] W_p^T, in fp32 throughout and with
-// the row maxima of |x_p| on the way.  A product's sum is a chain of its own, as of one linear after the other.  128 (64) rows a
-// workgroup, slabs of 32 k in two LDS buffers with the loads of the next two in flight; k pairs and strides as in linear_rows_kernel.
-// Five products of 256 channels, us here / in five launches of linear_kernel / bytes at 5 TB/s: 73 728 rows -> 16 109 / 200 / 76,
-// 24 576 -> 64 62 / 165 / 26.  Bound by the slab in turn: with one slab in flight 114 and 98.
+// the row maxima of |x_p| on the way.  A product's sum is a chain of its own, as of one linear after the other.  Slabs of 32 k in two
+// LDS buffers with the loads of the next two in flight; a wave has MB x NB blocks of B x B, a workgroup 16 to 128 columns of 32 or 64 rows.
+// Bound by the slab in turn (with one slab in flight half as fast) and, unevenly, by the matrix cores: blocks of 16 where there are few
+// columns, which leave none of them empty, and the row count that gives every CU its share.  Five products of 256 channels, us with
+// blocks of 16 / of 32 in tiles of 128 and 64 rows / in five launches of linear_kernel / bytes at 5 TB/s: 73 728 rows -> 16 85 / 104 /
+// 200 / 76, 18 432 29 / 42, 3000 22 / 40; 24 576 -> 64 55 / 63 / 165 / 26, 900 26 / 37.  Beyond 64 columns the larger blocks read less
+// of LDS for what they multiply: 24 576 x 64 -> 256 20.5 against 23.8.  The error against float64 is the same, 2.9e-7.
 struct ProductWeights { const float* W[kMaxProducts]; };
-template <int WAVES_M, int NI>
+template <int B, int WAVES_M, int MB, int NB>
 __global__ void __launch_bounds__(256)
 linear_products_kernel(const ProductWeights weights, long so, const float* __restrict__ X, long R, int C, int G, int O,
                        float* __restrict__ Y, float* __restrict__ xmax, int tiles_n, long tiles_total) {
-    constexpr int WAVES_N = 4 / WAVES_M, TM = 32 * WAVES_M, TN = 32 * NI * WAVES_N, XL = TM / 32, WL = TN / 32;
+    constexpr int WAVES_N = 4 / WAVES_M, TM = B * MB * WAVES_M, TN = B * NB * WAVES_N, XL = TM / 32, WL = TN < 32 ? 1 : TN / 32;
+    constexpr int kRun = B / 2, kRegs = B * B / 64;           // k's of a lane in a slab, registers of a block
+    typedef float Block __attribute__((ext_vector_type(kRegs)));
+    static_assert(TM % 32 == 0 && (TN == 16 || TN % 32 == 0), "32 rows of a slab at a time");
     __shared__ __attribute__((aligned(16))) float xs[2][TM * kRS1];
-    __shared__ __attribute__((aligned(16))) float ws[2][TN * kRS1];
+    __shared__ __attribute__((aligned(16))) float ws[2][32 * WL * kRS1];
     // XCD-aware tile order
     const long per_xcd = (tiles_total + 7) / 8, logical = (long)(blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (logical >= tiles_total) return;
     const long tile_m = logical / tiles_n;
     const int tile_n = (int)(logical - tile_m * tiles_n);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, khalf = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, part = lane / B;
     const int wave_m = wave / WAVES_N, wave_n = wave % WAVES_N;
     const long r0 = tile_m * TM, row_floats = (long)G * C;
     const int n0 = tile_n * TN;
@@ -437,15 +443,17 @@ linear_products_kernel(const ProductWeights weights, long so, const float* __res
         c_load = last ? c_load : (next ? 0 : c_load + 1);
         p_load += next && !last ? 1 : 0;
     };
-    float16v acc[NI], sum[NI];
+    Block acc[MB][NB], sum[MB][NB];
 #pragma unroll
-    for (int ni = 0; ni < NI; ni++)
+    for (int mb = 0; mb < MB; mb++)
 #pragma unroll
-        for (int q = 0; q < 16; q++) acc[ni][q] = sum[ni][q] = 0.f;
+        for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+            for (int q = 0; q < kRegs; q++) acc[mb][nb][q] = sum[mb][nb][q] = 0.f;
     float mx[XL];
 #pragma unroll
     for (int j = 0; j < XL; j++) mx[j] = 0.f;
-    const int a_off = (wave_m * 32 + (lane & 31)) * kRS1 + khalf * 16, b_off = (wave_n * NI * 32 + (lane & 31)) * kRS1 + khalf * 16;
+    const int a_off = (wave_m * B * MB + lane % B) * kRS1 + part * kRun, b_off = (wave_n * B * NB + lane % B) * kRS1 + part * kRun;
 
     int p = 0, c = 0;                                         // the slab to be multiplied
     auto step = [&](Slab& v, float* xb, float* wb) __attribute__((always_inline)) {
@@ -459,29 +467,36 @@ linear_products_kernel(const ProductWeights weights, long so, const float* __res
         __syncthreads();                                      // (this buffer is written again behind the next of these)
         load(v);
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int half = 0; half < 2; half++) {
-            float a[8], b[NI][8];
+        auto read = [&](const float* from, float (&to)[8]) {
 #pragma unroll
             for (int k = 0; k < 2; k++) {
-                const float4 t = *reinterpret_cast<const float4*>(xb + a_off + half * 8 + 4 * k);
-                a[4 * k] = t.x; a[4 * k + 1] = t.y; a[4 * k + 2] = t.z; a[4 * k + 3] = t.w;
-#pragma unroll
-                for (int ni = 0; ni < NI; ni++) {
-                    const float4 u = *reinterpret_cast<const float4*>(wb + b_off + 32 * ni * kRS1 + half * 8 + 4 * k);
-                    b[ni][4 * k] = u.x; b[ni][4 * k + 1] = u.y; b[ni][4 * k + 2] = u.z; b[ni][4 * k + 3] = u.w;
-                }
+                const float4 t = *reinterpret_cast<const float4*>(from + 4 * k);
+                to[4 * k] = t.x; to[4 * k + 1] = t.y; to[4 * k + 2] = t.z; to[4 * k + 3] = t.w;
             }
+        };
+#pragma unroll
+        for (int at = 0; at < kRun; at += 8) {
+            float a[MB][8], b[NB][8];
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) read(xb + a_off + B * mb * kRS1 + at, a[mb]);
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++) read(wb + b_off + B * nb * kRS1 + at, b[nb]);
 #pragma unroll
             for (int k = 0; k < 8; k++)
 #pragma unroll
-                for (int ni = 0; ni < NI; ni++) acc[ni] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[k], b[ni][k], acc[ni], 0, 0, 0);
+                for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+                    for (int nb = 0; nb < NB; nb++)
+                        if constexpr (B == 16) acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[mb][k], b[nb][k], acc[mb][nb], 0, 0, 0);
+                        else acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[mb][k], b[nb][k], acc[mb][nb], 0, 0, 0);
         }
         if (++c < slabs) return;
 #pragma unroll
-        for (int ni = 0; ni < NI; ni++)
+        for (int mb = 0; mb < MB; mb++)
 #pragma unroll
-            for (int q = 0; q < 16; q++) { sum[ni][q] += acc[ni][q]; acc[ni][q] = 0.f; }
+            for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+                for (int q = 0; q < kRegs; q++) { sum[mb][nb][q] += acc[mb][nb][q]; acc[mb][nb][q] = 0.f; }
 #pragma unroll
         for (int j = 0; j < XL; j++) {
             float m = mx[j];
@@ -503,24 +518,26 @@ linear_products_kernel(const ProductWeights weights, long so, const float* __res
     }
     if (total_slabs & 1) step(even, xs[0], ws[0]);
 #pragma unroll
-    for (int ni = 0; ni < NI; ni++) {
-        const int n = n0 + (wave_n * NI + ni) * 32 + (lane & 31);
+    for (int nb = 0; nb < NB; nb++) {
+        const int n = n0 + (wave_n * NB + nb) * B + lane % B;
         if (n >= O) continue;
 #pragma unroll
-        for (int q = 0; q < 16; q++) {
-            const long r = r0 + wave_m * 32 + 8 * (q / 4) + 4 * khalf + (q % 4);
-            if (r < R) Y[r * O + n] = sum[ni][q];
-        }
+        for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+            for (int q = 0; q < kRegs; q++) {
+                const long r = r0 + (wave_m * MB + mb) * B + B / 4 * (q / 4) + 4 * part + q % 4;
+                if (r < R) Y[r * O + n] = sum[mb][nb][q];
+            }
     }
 }
 
-template <int WAVES_M, int NI>
+template <int B, int WAVES_M, int MB, int NB>
 int launch_products(const ProductWeights& weights, long so, const float* X, long R, int C, int G, int O, float* Y, float* xmax,
                     hipStream_t st) {
-    const int tiles_n = (int)ceil_div(O, 32 * NI * (4 / WAVES_M));
-    const long total = ceil_div(R, 32 * WAVES_M) * tiles_n, grid = ceil_div(total, 8) * 8;
+    const int tiles_n = (int)ceil_div(O, B * NB * (4 / WAVES_M));
+    const long total = ceil_div(R, B * MB * WAVES_M) * tiles_n, grid = ceil_div(total, 8) * 8;
     MG_REQUIRE(grid <= 0x7fffffffL, "mg_tensor_linear_products: grid too large (rows=%ld dim_out=%d)", R, O);
-    hipLaunchKernelGGL((linear_products_kernel<WAVES_M, NI>), dim3((unsigned)grid), dim3(256), 0, st, weights, so, X, R, C, G, O, Y, xmax,
+    hipLaunchKernelGGL((linear_products_kernel<B, WAVES_M, MB, NB>), dim3((unsigned)grid), dim3(256), 0, st, weights, so, X, R, C, G, O, Y, xmax,
                        tiles_n, total);
     return check_launch("mg_tensor_linear_products");
 }
@@ -846,9 +863,11 @@ int mg_tensor_linear_products(const float* const* W, long w_stride_o, int produc
         weights.W[p] = W[p];
     }
     hipStream_t st = (hipStream_t)stream;
-    if (dim_out <= 32) return launch_products<4, 1>(weights, w_stride_o, x, rows, dim_in, products, dim_out, y, x_rowmax, st);
-    if (dim_out <= 64) return launch_products<2, 1>(weights, w_stride_o, x, rows, dim_in, products, dim_out, y, x_rowmax, st);
-    return launch_products<2, 2>(weights, w_stride_o, x, rows, dim_in, products, dim_out, y, x_rowmax, st);
+    auto run = [&](auto launch) { return launch(weights, w_stride_o, x, rows, dim_in, products, dim_out, y, x_rowmax, st); };
+    if (dim_out <= 16) return run(launch_products<16, 4, 1, 1>);
+    if (dim_out <= 32) return run(launch_products<16, 4, 1, 2>);
+    if (dim_out <= 64) return run(launch_products<16, 2, 1, 2>);
+    return run(launch_products<32, 2, 1, 2>);
 }
 
 int mg_set_linear_mode(int mode) {

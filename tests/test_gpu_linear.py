@@ -981,3 +981,23 @@ def test_reductions_split_over_waves_with_one_chunk_and_several(ops, rows, dim_i
     keep = torch.ones(nodes, dtype=torch.bool, device="cuda")
     keep[rows // 2 // comps] = False
     assert torch.equal(z[keep], y[keep])
+
+
+@pytest.mark.parametrize("rows, products, dim_in, dim_out", [
+    (1, 1, 32, 1), (33, 5, 64, 16), (64, 2, 96, 17), (95, 8, 32, 32), (31, 3, 160, 33), (2049, 5, 256, 64), (65, 4, 64, 65), (130, 2, 32, 130)])
+def test_linears_side_by_side_at_the_edges_of_their_tiles(ops, rows, products, dim_in, dim_out):
+    """Both block sizes and each tile: rows and columns that end inside one, an odd number of slabs.  In fp32: every addition of a chain of
+    dim_in products, and of the products' sums, rounds by 2^-24 of at most the norms of what is multiplied.  Row maxima are exact, and a
+    row does not depend on those beside it."""
+    g = torch.Generator().manual_seed(rows + dim_out)
+    x = torch.randn(rows, products * dim_in, generator=g).cuda()
+    W = [torch.randn(dim_out, dim_in, generator=g).cuda() for _ in range(products)]
+    y, m = ops.row_linears_fwd(x, W, 9, True)
+    parts = x.double().view(rows, products, dim_in)
+    ref = sum(parts[:, k] @ W[k].double().t() for k in range(products))
+    size = sum(parts[:, k].norm(dim=1)[:, None] * W[k].double().norm(dim=1) for k in range(products))
+    assert float(((y.double() - ref).abs() / size).max()) <= (dim_in + products) * 2.0 ** -24
+    assert torch.equal(m, x.view(rows, products, dim_in).abs().amax(2))
+    x[0] = float("inf")
+    z, _ = ops.row_linears_fwd(x, W, 9, True)
+    assert torch.equal(z[1:], y[1:]) and not bool(z[0].isfinite().any())
