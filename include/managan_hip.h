@@ -1070,6 +1070,10 @@ int mg_bee_node_products(long n_nodes, int chan, const float* l0, const float* l
 int mg_bee_node_products_grad(long n_nodes, int chan, const float* l0, const float* l1, const float* l2, const float* r0,
                               const float* r1, const float* r2, const float* d_P0, const float* d_P1, const float* d_P2,
                               float* g_l0, float* g_l1, float* g_l2, float* g_r0, float* g_r1, float* g_r2, mg_stream_t stream);
+/* The same where the rank-2 products have no gradient. */
+int mg_bee_node_products_grad_lower(long n_nodes, int chan, const float* l0, const float* l1, const float* l2, const float* r0,
+                                    const float* r1, const float* r2, const float* d_P0, const float* d_P1, float* g_l0, float* g_l1,
+                                    float* g_l2, float* g_r0, float* g_r1, float* g_r2, mg_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * bf16-storage configuration: feature tensors are bf16 in memory (void* below), every

@@ -122,6 +122,7 @@ _SIGNATURES = {
     "mg_radial_encode": [i32, vp, i64, i32, f32, vp, vp],
     "mg_bee_node_products": [i64, i32, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp],
     "mg_bee_node_products_grad": [i64, i32] + [vp] * 16,
+    "mg_bee_node_products_grad_lower": [i64, i32] + [vp] * 15,
     "mg_bee_node_products_bf16": [i64, i32, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp],
     "mg_tensor_linear_bf16": [vp, vp, i64, i32, i32, vp, i32, i32, i32, i32, vp, vp],
     "mg_bee_message_bf16": [vp, vp, vp, i32, i64, vp, vp, vp, vp, vp, i32, vp, vp, vp, vp, vp, vp],

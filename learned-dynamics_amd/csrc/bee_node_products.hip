@@ -90,7 +90,9 @@ __global__ void __launch_bounds__(256) node_products_kernel(long n_nodes, int ch
 
 // The adjoint on the same rows: both operands' gradients in one pass, a lane per (node, channel), 26 operand and 63 gradient values
 // in, 26 out: bound by HBM (8192 rows, 256 channels: 0.21 ms, 4.6 TB/s).  With a kernel an operand on (row, chan, comp) arrays 0.32 ms,
-// and the gradients of 13 linears to transpose before and after.
+// and the gradients of 13 linears to transpose before and after.  WITH_P2 false: the rank-2 products lead nowhere (the last block of a
+// denoiser, whose rank-2 features are not read), and 45 of the 63 gradients are no zeros to be written first and read here (8192 rows with the writing of the zeros 270 -> 110 us).
+template <bool WITH_P2>
 __global__ void __launch_bounds__(256) node_products_grad_kernel(long n_nodes, int chan, const float* __restrict__ l0,
                                                                  const float* __restrict__ l1, const float* __restrict__ l2,
                                                                  const float* __restrict__ r0, const float* __restrict__ r1,
@@ -152,6 +154,7 @@ __global__ void __launch_bounds__(256) node_products_grad_kernel(long n_nodes, i
         gv[0] += q111[1] * u[2] - q111[2] * u[1];
         gv[1] += q111[2] * u[0] - q111[0] * u[2];
         gv[2] += q111[0] * u[1] - q111[1] * u[0];
+        if constexpr (WITH_P2)
 #pragma unroll
         for (int x = 0; x < 3; x++) {
             float h[3];
@@ -380,6 +383,22 @@ int launch(const char* what, long n_nodes, int chan, const void* l0, const void*
 
 using namespace mg;
 
+namespace {
+template <bool WITH_P2>
+int node_products_grad(long n_nodes, int chan, const float* l0, const float* l1, const float* l2, const float* r0, const float* r1,
+                       const float* r2, const float* d_P0, const float* d_P1, const float* d_P2, float* g_l0, float* g_l1, float* g_l2,
+                       float* g_r0, float* g_r1, float* g_r2, mg_stream_t stream) {
+    MG_REQUIRE(n_nodes >= 0 && chan > 0, "mg_bee_node_products_grad: bad size");
+    if (n_nodes == 0) return MG_OK;
+    MG_REQUIRE(l0 && l1 && l2 && r0 && r1 && r2 && d_P0 && d_P1 && g_l0 && g_l1 && g_l2 && g_r0 && g_r1 && g_r2,
+               "mg_bee_node_products_grad: null pointer");
+    const long blocks = ceil_div(n_nodes * chan, 256);
+    hipLaunchKernelGGL(node_products_grad_kernel<WITH_P2>, dim3((unsigned)(blocks < 65536 ? blocks : 65536)), dim3(256), 0,
+                       (hipStream_t)stream, n_nodes, chan, l0, l1, l2, r0, r1, r2, d_P0, d_P1, d_P2, g_l0, g_l1, g_l2, g_r0, g_r1, g_r2);
+    return check_launch("mg_bee_node_products_grad");
+}
+}  // namespace
+
 extern "C" {
 
 int mg_bee_node_products(long n_nodes, int chan, const float* l0, const float* l1, const float* l2, const float* r0,
@@ -391,14 +410,14 @@ int mg_bee_node_products(long n_nodes, int chan, const float* l0, const float* l
 int mg_bee_node_products_grad(long n_nodes, int chan, const float* l0, const float* l1, const float* l2, const float* r0,
                               const float* r1, const float* r2, const float* d_P0, const float* d_P1, const float* d_P2,
                               float* g_l0, float* g_l1, float* g_l2, float* g_r0, float* g_r1, float* g_r2, mg_stream_t stream) {
-    MG_REQUIRE(n_nodes >= 0 && chan > 0, "mg_bee_node_products_grad: bad size");
-    if (n_nodes == 0) return MG_OK;
-    MG_REQUIRE(l0 && l1 && l2 && r0 && r1 && r2 && d_P0 && d_P1 && d_P2 && g_l0 && g_l1 && g_l2 && g_r0 && g_r1 && g_r2,
-               "mg_bee_node_products_grad: null pointer");
-    const long blocks = ceil_div(n_nodes * chan, 256);
-    hipLaunchKernelGGL(node_products_grad_kernel, dim3((unsigned)(blocks < 65536 ? blocks : 65536)), dim3(256), 0, (hipStream_t)stream,
-                       n_nodes, chan, l0, l1, l2, r0, r1, r2, d_P0, d_P1, d_P2, g_l0, g_l1, g_l2, g_r0, g_r1, g_r2);
-    return check_launch("mg_bee_node_products_grad");
+    MG_REQUIRE(n_nodes <= 0 || d_P2, "mg_bee_node_products_grad: null pointer");
+    return node_products_grad<true>(n_nodes, chan, l0, l1, l2, r0, r1, r2, d_P0, d_P1, d_P2, g_l0, g_l1, g_l2, g_r0, g_r1, g_r2, stream);
+}
+
+int mg_bee_node_products_grad_lower(long n_nodes, int chan, const float* l0, const float* l1, const float* l2, const float* r0,
+                                    const float* r1, const float* r2, const float* d_P0, const float* d_P1, float* g_l0, float* g_l1,
+                                    float* g_l2, float* g_r0, float* g_r1, float* g_r2, mg_stream_t stream) {
+    return node_products_grad<false>(n_nodes, chan, l0, l1, l2, r0, r1, r2, d_P0, d_P1, nullptr, g_l0, g_l1, g_l2, g_r0, g_r1, g_r2, stream);
 }
 
 int mg_bee_node_products_rank2(long n_nodes, int chan, const float* l0, const float* l1, const float* l2,

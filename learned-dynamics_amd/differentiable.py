@@ -1172,8 +1172,9 @@ class _NodeProducts(torch.autograd.Function):
         else:
             N, C = operands[0].shape
             shapes = (N, 3, C), (N, 3, 5, C), (N, 9, 5, C)
-            grads = ops.bee_node_products_grad(operands, [operands[0].new_zeros(sh) if g is None else g.contiguous()
-                                                          for g, sh in zip(dys, shapes)])
+            # (without a gradient of P2, 45 of a node's 63, none is written as zeros to be read)
+            grads = ops.bee_node_products_grad(operands, [g if g is None and k == 2 else operands[0].new_zeros(sh) if g is None else g.contiguous()
+                                                          for k, (g, sh) in enumerate(zip(dys, shapes))])
         return tuple(g if nd else None for g, nd in zip(grads, need))
 
 

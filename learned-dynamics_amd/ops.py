@@ -1381,18 +1381,20 @@ def bee_node_products(l0, l1, l2, r0, r1, r2, want_node_max=False):
 
 
 def bee_node_products_grad(operands, d_products):
-    """The gradients of bee_node_products (float32) for its six operands from those of P0, P1, P2."""
+    """The gradients of bee_node_products (float32) for its six operands from those of P0, P1, P2; the last may be None: P2 leads nowhere."""
     l0 = operands[0]
+    d_products = [t for k, t in enumerate(d_products) if k < 2 or t is not None]
     for t in (*operands, *d_products):
         _check_input(t, "operand or gradient")
     N, chan = int(l0.size(0)), int(l0.size(1))
     if [t.numel() for t in operands] != 2 * [N * chan, 3 * N * chan, 9 * N * chan]:
         raise RuntimeError("operands must be (nodes, chan), (nodes, 3, chan), (nodes, 9, chan)")
-    if [t.numel() for t in d_products] != [3 * N * chan, 15 * N * chan, 45 * N * chan]:
+    if len(d_products) < 2 or [t.numel() for t in d_products] != [3 * N * chan, 15 * N * chan, 45 * N * chan][:len(d_products)]:
         raise RuntimeError("gradients must have the sizes of P0, P1, P2")
+    run = _lib.mg_bee_node_products_grad if len(d_products) == 3 else _lib.mg_bee_node_products_grad_lower
     with _on(l0.device):
         grads = [torch.empty_like(t) for t in operands]
-        L.check(_lib.mg_bee_node_products_grad(N, chan, *[_p(t) for t in (*operands, *d_products, *grads)], _stream()))
+        L.check(run(N, chan, *[_p(t) for t in (*operands, *d_products, *grads)], _stream()))
     return grads
 
 
