@@ -400,3 +400,23 @@ def test_tens_group_norm_bf16_where_columns_and_threads_do_not_divide(ops, comps
     """Rows that leave threads of the statistics pass without a column (a row of one 16-byte piece, of 15), groups that 256
     threads do not divide by, one thread to a group, and one piece more than a workgroup has threads."""
     test_tens_group_norm_bf16(ops, comps, chan, groups, False)
+
+
+@pytest.mark.parametrize("rows", [1, 129, 4099])
+def test_sums_of_the_scalar_chain_as_one_operand(ops, rows):
+    """The sums side by side are those of the two results, rounded to bfloat16 to the bit; the counted bias; segments that are empty, end
+    inside a block of 32 rows and span several."""
+    g = torch.Generator().manual_seed(rows)
+    lengths = torch.tensor([0, 1, 30, 1, 0, 3, 100, 29, 0])
+    ends = torch.cat([lengths, torch.randint(0, 50, (rows // 20 + 4,), generator=g)]).cumsum(0).clamp(max=rows)
+    ends[-1] = rows
+    row_ptr = torch.cat([torch.zeros(1, dtype=torch.long), ends])
+    seg = torch.repeat_interleave(torch.arange(ends.numel()), row_ptr.diff()).int().cuda()
+    x = torch.randn(rows, 64, generator=g).cuda().to(torch.bfloat16)
+    Y, W1, W2 = ((torch.randn(o, k, generator=g) / k ** 0.5).cuda() for o, k in ((128, 64), (256, 128), (256, 256)))
+    b1, b2, bias = (torch.randn(n, generator=g).cuda() for n in (256, 256, 128))
+    args = (Y, x, W1, b1, W2, b2, row_ptr.int().cuda(), seg, ends.numel())
+    s_psi, s_h = ops.mlp_chain_bf16(*args)
+    sums, base = ops.mlp_chain_bf16(*args, count_bias=bias)
+    assert torch.equal(sums, torch.cat([s_h, s_psi], 1).to(torch.bfloat16))
+    assert torch.equal(base, row_ptr.diff().float().cuda()[:, None] * bias)
