@@ -639,7 +639,7 @@ std::tuple<at::Tensor, at::Tensor> painn_update(const at::Tensor& x_a, const at:
     if (n <= 256) cat_max = floats(x_a, {rows, 1});
     const mg_stream_t st = stream_of(x_a);
     // the rows and widths whose component linear is the split-fp16 one (figures at the kernel)
-    const bool maps = mg_get_linear_mode() == kModeF16x2 && rows >= (n <= 224 ? 1280 : 2304) && packs_f16x2(W_lrv) &&
+    const bool maps = mg_get_linear_mode() == kModeF16x2 && rows >= (n <= 128 ? 1 : n <= 224 ? 1280 : 2304) && packs_f16x2(W_lrv) &&
                       mg_painn_update_maps_supported((int)n) && aligned16(x_v) && aligned16(x_a);
     if (maps) {
         lrv = floats(x_a, {rows, 3, n});
