@@ -124,8 +124,8 @@ def messages_forward(mod: Messages, graph: Graph, r_ij, s_a, s_v, s_d, node_orde
     Ls = mod.mlp_a.layers
     if chain and ops.mlp_chain_bf16_supported(E, 3 * chan, Y0.shape[0], Ls[0].out_features) \
             and Ls[2].out_features == Ls[0].out_features:
-        # psi_a and both hidden layers stay in registers; only their sums over the edges of a node are written
-        # (W_last | W_direct + 1) on them side by side, the scale in the weights: one linear
+        # psi_a and both hidden layers stay on chip, only their sums over the edges of a node are written; (W_last | W_direct + 1)
+        # on these side by side, the scale in the weights: one linear
         direct, last = mod.mlp_a.lin_direct.weight, Ls[4]
         tail, bias = _derived(mod.mlp_a, "tail_of_sums", (direct, last.weight, last.bias), lambda: (
             0.1 * torch.cat((last.weight, direct + torch.eye(direct.shape[0], device=direct.device, dtype=direct.dtype)), 1),
