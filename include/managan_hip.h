@@ -874,13 +874,6 @@ int mg_mlp_chain_bf16_workspace_bytes(long rows, size_t* bytes);
 int mg_mlp_chain_bf16(const void* x, long rows, int dim_in, const void* packed_Y, const void* packed_W1,
                       const float* b1, const void* packed_W2, const float* b2, int act, const int* row_ptr,
                       const int* seg, long n_out, void* workspace, float* sum_psi, float* sum_h2, mg_stream_t stream);
-/* The same with the sums as the operand of the linears behind them: sums (n_out, 384) bfloat16 takes those of h2 and then of psi,
- * base (n_out, 128) the rows of the segment times count_bias (128).  sum_psi and sum_h2 are then room for the rows of segments that
- * end inside a block of 32 rows, not results. */
-int mg_mlp_chain_bf16_sums(const void* x, long rows, int dim_in, const void* packed_Y, const void* packed_W1, const float* b1,
-                           const void* packed_W2, const float* b2, int act, const int* row_ptr, const int* seg, long n_out,
-                           void* workspace, float* sum_psi, float* sum_h2, const float* count_bias, float* base, void* sums,
-                           mg_stream_t stream);
 
 /* The three edge sums of DisplacementTensors.forward (archs/diffuser_atoms15.py:218-224) over CSR rows: with
  * u = s r / sqrt(1 + |s r|^2), s = scale (7 / r0 in the reference, tens_sigmoid of managan/tensor_products.py:167-182),

@@ -124,15 +124,10 @@ def messages_forward(mod: Messages, graph: Graph, r_ij, s_a, s_v, s_d, node_orde
     Ls = mod.mlp_a.layers
     if chain and ops.mlp_chain_bf16_supported(E, 3 * chan, Y0.shape[0], Ls[0].out_features) \
             and Ls[2].out_features == Ls[0].out_features:
-        # psi_a and both hidden layers stay on chip, only their sums over the edges of a node are written; (W_last | W_direct + 1)
-        # on these side by side, the scale in the weights: one linear
-        direct, last = mod.mlp_a.lin_direct.weight, Ls[4]
-        tail, bias = _derived(mod.mlp_a, "tail_of_sums", (direct, last.weight, last.bias), lambda: (
-            0.1 * torch.cat((last.weight, direct + torch.eye(direct.shape[0], device=direct.device, dtype=direct.dtype)), 1),
-            0.1 * last.bias))
-        sums, out = ops.mlp_chain_bf16(Y0, P0.reshape(E, 3 * chan), Ls[0].weight, Ls[0].bias, Ls[2].weight, Ls[2].bias, graph.row_ptr,
-                                       graph.src32, rows, count_bias=bias)
-        B_a = ops.tensor_linear_bf16(tail, sums, out=out, accumulate=True).to(torch.bfloat16)
+        # psi_a and both hidden layers stay on chip; only their sums over the edges of a node are written
+        s_psi, s_h = ops.mlp_chain_bf16(Y0, P0.reshape(E, 3 * chan), Ls[0].weight, Ls[0].bias, Ls[2].weight,
+                                        Ls[2].bias, graph.row_ptr, graph.src32, rows)
+        B_a = _mlp_after_sums(mod.mlp_a, s_psi.to(torch.bfloat16), s_h.to(torch.bfloat16), graph.row_ptr, True, 0.1)
     else:
         if ops.bf16_rowsum_supported(E, 3 * chan, Y0.shape[0]):
             s_psi, psi_a = ops.tensor_linear_bf16_rowsum(Y0, P0.reshape(E, 3 * chan), graph.row_ptr, graph.src32,

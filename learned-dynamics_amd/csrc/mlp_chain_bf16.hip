@@ -280,40 +280,6 @@ mlp_chain_bf16_kernel(const __bf16* __restrict__ X, long R, int I, const __bf16*
     }
 }
 
-// What rowsum_finish_kernel does to both sums, in one launch and as the operand of the linears behind them: S (n_out, 384) takes the sums
-// of h2 and then of psi, rounded to bfloat16; base (n_out, 128) the rows of the segment times bias, which those linears add to.
-// (Two finishing launches, two roundings, the rows' count and the bias's addition were eight.)
-constexpr int kSumQuads = (kD + kH) / 4;
-__global__ void __launch_bounds__(256)
-mlp_chain_finish_kernel(const int* __restrict__ row_ptr, long n_out, long n_blocks, const float* __restrict__ slots_x,
-                        const float* __restrict__ slots_h, const float* __restrict__ sum_psi, const float* __restrict__ sum_h,
-                        const float* __restrict__ bias, float* __restrict__ base, __bf16* __restrict__ S) {
-    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n_out * kSumQuads) return;
-    const long s_id = idx / kSumQuads;
-    const int quad = (int)(idx - s_id * kSumQuads);
-    const bool psi = quad >= kH / 4;
-    const int O = psi ? kD : kH, x = 4 * (psi ? quad - kH / 4 : quad);
-    const float* const slots = psi ? slots_x : slots_h;
-    const long lo = row_ptr[s_id], hi = row_ptr[s_id + 1], b_lo = lo / 32, b_hi = (hi - 1) / 32;
-    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (hi > lo && b_lo == b_hi && lo > 32 * b_lo && hi - 1 < 32 * b_lo + 31) {
-        s = *reinterpret_cast<const float4*>((psi ? sum_psi : sum_h) + s_id * O + x);      // written directly
-    } else if (hi > lo) {
-        for (long b = b_lo; b <= b_hi; b++) {
-            const float4 t = *reinterpret_cast<const float4*>(slots + (32 * b >= lo ? b : n_blocks + b) * O + x);
-            s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
-        }
-    }
-    typedef __bf16 Four __attribute__((ext_vector_type(4)));
-    *reinterpret_cast<Four*>(S + s_id * (kD + kH) + 4 * quad) = Four{(__bf16)s.x, (__bf16)s.y, (__bf16)s.z, (__bf16)s.w};
-    if (psi) {
-        const float count = (float)(hi - lo);
-        const float4 c = *reinterpret_cast<const float4*>(bias + x);
-        *reinterpret_cast<float4*>(base + s_id * kD + x) = make_float4(count * c.x, count * c.y, count * c.z, count * c.w);
-    }
-}
-
 }  // namespace
 }  // namespace mg
 
@@ -324,9 +290,15 @@ static long chain_weight_elems(int dim_in) { return 2L * kH * kD + 2L * kH * kH 
 
 extern "C" {
 
-static int mlp_chain(const void* x, long rows, int dim_in, const void* packed_Y, const void* packed_W1, const float* b1,
-                     const void* packed_W2, const float* b2, int act, const int* row_ptr, const int* seg, long n_out, void* workspace,
-                     float* sum_psi, float* sum_h2, const float* count_bias, float* base, void* sums, mg_stream_t stream) {
+int mg_mlp_chain_bf16_workspace_bytes(long rows, size_t* bytes) {
+    MG_REQUIRE(bytes != nullptr && rows >= 0, "mg_mlp_chain_bf16_workspace_bytes: bad argument");
+    *bytes = (size_t)(2L * (ceil_div(rows, 32) + 1) * (kD + kH)) * sizeof(float) + chain_weight_elems(kPackedDimIn) * sizeof(__bf16);
+    return MG_OK;
+}
+
+int mg_mlp_chain_bf16(const void* x, long rows, int dim_in, const void* packed_Y, const void* packed_W1,
+                      const float* b1, const void* packed_W2, const float* b2, int act, const int* row_ptr,
+                      const int* seg, long n_out, void* workspace, float* sum_psi, float* sum_h2, mg_stream_t stream) {
     MG_REQUIRE(dim_in >= 32 && dim_in % 32 == 0, "mg_mlp_chain_bf16: dim_in must be a multiple of 32 (got %d)", dim_in);
     MG_REQUIRE(rows >= 0 && n_out >= 0 && rows < (1L << 31) && n_out < (1L << 31), "mg_mlp_chain_bf16: bad size");
     MG_REQUIRE(act >= 0 && act <= 2, "mg_mlp_chain_bf16: unknown activation %d", act);
@@ -365,40 +337,12 @@ static int mlp_chain(const void* x, long rows, int dim_in, const void* packed_Y,
         else planes ? launch(mlp_chain_bf16_kernel<0, true>) : launch(mlp_chain_bf16_kernel<0, false>);
         if (int code = check_launch("mlp_chain_bf16_kernel")) return code;
     }
-    if (sums) {
-        mlp_chain_finish_kernel<<<dim3((unsigned)ceil_div(n_out * kSumQuads, 256)), dim3(256), 0, st>>>(
-            row_ptr, n_out, n_blocks, slots_x, slots_h, sum_psi, sum_h2, count_bias, base, static_cast<__bf16*>(sums));
-        return check_launch("mlp_chain_finish_kernel");
-    }
     rowsum_finish_kernel<<<dim3((unsigned)ceil_div(n_out * (kD / 4), 256)), dim3(256), 0, st>>>(
         row_ptr, n_out, n_blocks, kD, slots_x, 1.0f, sum_psi);
     if (int code = check_launch("rowsum_finish_kernel")) return code;
     rowsum_finish_kernel<<<dim3((unsigned)ceil_div(n_out * (kH / 4), 256)), dim3(256), 0, st>>>(
         row_ptr, n_out, n_blocks, kH, slots_h, 1.0f, sum_h2);
     return check_launch("rowsum_finish_kernel");
-}
-
-int mg_mlp_chain_bf16_workspace_bytes(long rows, size_t* bytes) {
-    MG_REQUIRE(bytes != nullptr && rows >= 0, "mg_mlp_chain_bf16_workspace_bytes: bad argument");
-    *bytes = (size_t)(2L * (ceil_div(rows, 32) + 1) * (kD + kH)) * sizeof(float) + chain_weight_elems(kPackedDimIn) * sizeof(__bf16);
-    return MG_OK;
-}
-
-int mg_mlp_chain_bf16(const void* x, long rows, int dim_in, const void* packed_Y, const void* packed_W1,
-                      const float* b1, const void* packed_W2, const float* b2, int act, const int* row_ptr,
-                      const int* seg, long n_out, void* workspace, float* sum_psi, float* sum_h2, mg_stream_t stream) {
-    return mlp_chain(x, rows, dim_in, packed_Y, packed_W1, b1, packed_W2, b2, act, row_ptr, seg, n_out, workspace, sum_psi, sum_h2,
-                     nullptr, nullptr, nullptr, stream);
-}
-
-int mg_mlp_chain_bf16_sums(const void* x, long rows, int dim_in, const void* packed_Y, const void* packed_W1, const float* b1,
-                           const void* packed_W2, const float* b2, int act, const int* row_ptr, const int* seg, long n_out,
-                           void* workspace, float* sum_psi, float* sum_h2, const float* count_bias, float* base, void* sums,
-                           mg_stream_t stream) {
-    MG_REQUIRE(n_out <= 0 || (count_bias && base && sums && aligned16(count_bias) && aligned16(base) && aligned16(sums)),
-               "mg_mlp_chain_bf16_sums: null or unaligned operand");
-    return mlp_chain(x, rows, dim_in, packed_Y, packed_W1, b1, packed_W2, b2, act, row_ptr, seg, n_out, workspace, sum_psi, sum_h2,
-                     count_bias, base, sums, stream);
 }
 
 }  // extern "C"

@@ -1433,13 +1433,11 @@ def mlp_chain_bf16_supported(rows, dim_in, dim_psi, hidden):
     return dim_psi == 128 and hidden == 256 and dim_in % 32 == 0 and rows >= 4096
 
 
-def mlp_chain_bf16(Y, x, W1, b1, W2, b2, row_ptr, seg, n_out, act=ACT_LEAKY, count_bias=None):
+def mlp_chain_bf16(Y, x, W1, b1, W2, b2, row_ptr, seg, n_out, act=ACT_LEAKY):
     """(sum_psi (n_out, 128), sum_h2 (n_out, 256)) float32: the sums over the rows of each segment of the
     bfloat16-rounded psi = Y x and h2 = act(b2 + W2 act(b1 + W1 psi)), every layer rounded to bfloat16 as
     tensor_linear_bf16 stores it, in one kernel that writes no per-row tensor.  x (rows, dim_in) bfloat16 sorted
-    by segment (seg ascending, row_ptr its CSR form); Y (128, dim_in), W1 (256, 128), W2 (256, 256) float32.
-    count_bias (128): returns instead (sums, base) for the linears behind the sums: (n_out, 384) bfloat16, the sums of h2 and then of
-    psi, and (n_out, 128) float32, the rows of each segment times count_bias."""
+    by segment (seg ascending, row_ptr its CSR form); Y (128, dim_in), W1 (256, 128), W2 (256, 256) float32."""
     _check_bf16(x, "x")
     for t, nm in ((Y, "Y"), (W1, "W1"), (W2, "W2"), (b1, "b1"), (b2, "b2")):
         _check_input(t, nm)
@@ -1457,19 +1455,11 @@ def mlp_chain_bf16(Y, x, W1, b1, W2, b2, row_ptr, seg, n_out, act=ACT_LEAKY, cou
         s_psi = torch.empty(n_out, 128, dtype=torch.float32, device=x.device)
         s_h = torch.empty(n_out, 256, dtype=torch.float32, device=x.device)
         work = torch.empty(nbytes.value // 4, dtype=torch.float32, device=x.device)
-        args = (_p(x), rows, dim_in, _p(packed_weight(Y)), _p(packed_weight(_operand_order_columns(W1))), _p(b1),
-                _p(packed_weight(_operand_order_columns(W2))), _p(b2), int(act), _p(row_ptr), _p(seg), int(n_out), _p(work), _p(s_psi),
-                _p(s_h))
-        if count_bias is None:
-            L.check(_lib.mg_mlp_chain_bf16(*args, _stream()))
-            return s_psi, s_h
-        _check_input(count_bias, "count_bias")
-        if count_bias.numel() != 128:
-            raise RuntimeError("count_bias must have 128 elements")
-        sums = torch.empty(n_out, 384, dtype=torch.bfloat16, device=x.device)
-        base = torch.empty(n_out, 128, dtype=torch.float32, device=x.device)
-        L.check(_lib.mg_mlp_chain_bf16_sums(*args, _p(count_bias), _p(base), _p(sums), _stream()))
-    return sums, base
+        L.check(_lib.mg_mlp_chain_bf16(_p(x), rows, dim_in, _p(packed_weight(Y)),
+                                       _p(packed_weight(_operand_order_columns(W1))), _p(b1),
+                                       _p(packed_weight(_operand_order_columns(W2))), _p(b2), int(act), _p(row_ptr),
+                                       _p(seg), int(n_out), _p(work), _p(s_psi), _p(s_h), _stream()))
+    return s_psi, s_h
 
 
 def tens_group_norm_bf16_supported(comps, chan):

@@ -402,21 +402,31 @@ def test_tens_group_norm_bf16_where_columns_and_threads_do_not_divide(ops, comps
     test_tens_group_norm_bf16(ops, comps, chan, groups, False)
 
 
-@pytest.mark.parametrize("rows", [1, 129, 4099])
-def test_sums_of_the_scalar_chain_as_one_operand(ops, rows):
-    """The sums side by side are those of the two results, rounded to bfloat16 to the bit; the counted bias; segments that are empty, end
-    inside a block of 32 rows and span several."""
-    g = torch.Generator().manual_seed(rows)
-    lengths = torch.tensor([0, 1, 30, 1, 0, 3, 100, 29, 0])
-    ends = torch.cat([lengths, torch.randint(0, 50, (rows // 20 + 4,), generator=g)]).cumsum(0).clamp(max=rows)
-    ends[-1] = rows
-    row_ptr = torch.cat([torch.zeros(1, dtype=torch.long), ends])
-    seg = torch.repeat_interleave(torch.arange(ends.numel()), row_ptr.diff()).int().cuda()
-    x = torch.randn(rows, 64, generator=g).cuda().to(torch.bfloat16)
-    Y, W1, W2 = ((torch.randn(o, k, generator=g) / k ** 0.5).cuda() for o, k in ((128, 64), (256, 128), (256, 256)))
-    b1, b2, bias = (torch.randn(n, generator=g).cuda() for n in (256, 256, 128))
-    args = (Y, x, W1, b1, W2, b2, row_ptr.int().cuda(), seg, ends.numel())
-    s_psi, s_h = ops.mlp_chain_bf16(*args)
-    sums, base = ops.mlp_chain_bf16(*args, count_bias=bias)
-    assert torch.equal(sums, torch.cat([s_h, s_psi], 1).to(torch.bfloat16))
-    assert torch.equal(base, row_ptr.diff().float().cuda()[:, None] * bias)
+def test_scale_behind_the_summed_scalar_messages(pkg, ops):
+    """The 0.1 of the scalar messages is an fp32 product behind the linears on the sums, not rounded into their weights of 16 bits: with
+    W_direct + 1 the diagonal of bfloat16 numbers c and the last layer zero, c times the rounded sum of psi is exact in fp32 and the
+    increments are 0.1 times it rounded once more, to the bit."""
+    bl, b16, gl = (importlib.import_module(f"learned-dynamics_amd.{m}") for m in ("bee_layers", "bee_layers_bf16", "graph_layers"))
+    torch.manual_seed(4)
+    N, chan, r0 = 4096, 128, 5.0
+    side = (N / 0.1) ** (1 / 3)
+    mod = bl.Messages(r0, chan, chan, chan, chan).cuda()
+    x = torch.randn(1, N, chan), torch.randn(1, N, chan, 3), torch.randn(1, N, chan, 3, 3)
+    with torch.no_grad():
+        c = (1 + torch.rand(chan)).to(torch.bfloat16).float().cuda()
+        mod.mlp_a.lin_direct.weight.copy_(torch.diag(c - 1))
+        for p in (mod.mlp_a.layers[4].weight, mod.mlp_a.layers[4].bias):
+            p.zero_()
+        graph, r_ij = gl.graph_setup(r0, (side, side, side), (torch.rand(1, N, 3) * side).cuda(), neighbours_max=256, celllist_max=64)
+        s = b16.to_storage(*[t.cuda() for t in x])
+        got = b16.messages_forward(mod, graph, r_ij, *s)[0]
+        La, Lv, Ld = (ops.tensor_linear_bf16(W, t.reshape(-1, chan)).reshape(t.shape) for W, t in zip((mod.L0.W, mod.L1.W, mod.L2.W), s))
+        enc, rhat = ops.bee_edge_geometry(r_ij.contiguous(), r0)
+        P0 = ops.bee_message_bf16(graph.row_ptr, graph.dst32, rhat, enc, La, Lv, Ld, mod.lin_enc.weight, mod.lin_enc.bias,
+                                  node_order=getattr(graph, "cell_order", None))[0]
+        E, L = P0.shape[0], mod.mlp_a.layers
+        assert ops.mlp_chain_bf16_supported(E, 3 * chan, chan, L[0].out_features)
+        Y0 = torch.cat([getattr(mod, f"Y_{k}").W for k in bl.LABELS_0], 1)
+        s_psi, _ = ops.mlp_chain_bf16(Y0, P0.reshape(E, 3 * chan), L[0].weight, L[0].bias, L[2].weight, L[2].bias, graph.row_ptr,
+                                      graph.src32, N)
+    assert torch.equal(got, (s_psi.to(torch.bfloat16).float() * c * 0.1).to(torch.bfloat16))
