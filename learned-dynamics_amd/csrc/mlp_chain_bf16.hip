@@ -10,7 +10,7 @@
 // read them (fragment_at); a wave owns 32 output columns and reads the fragments of its weights straight from memory: a step of 16 k
 // is two contiguous kilobytes of the L2 and feeds eight matrix instructions, and no barrier stands in the loop over k of the hidden
 // layers.  Where rows are the first operand (psi, h2) a lane of the product holds rows of one column, which a segment's sum adds up in
-// a register; where they are the second (h1) four consecutive channels of one row, the next layer's operand eight bytes at a time.
+// a register; where they are the second (h1) channels of one row, the next layer's operand sixteen bytes at a time.
 //
 // 5.9 M rows of 384 with 90 to a segment 3.59 ms, 180 000 rows 0.125 ms; with psi, h1 and h2 in the registers of one wave per 32 rows
 // and the weights through LDS (two fragments read for two matrix instructions, a barrier for every 32 k) 4.11 and 0.134 ms.  What
@@ -25,7 +25,6 @@ namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kD = 128, kH = 256;
 constexpr int kBlocks = 4, kRows = 32 * kBlocks, kThreads = 512;  // row blocks and rows of a workgroup
@@ -47,13 +46,15 @@ __device__ __forceinline__ int piece_of(int k) { return ((k >> 3) & 1) + 2 * ((k
 __device__ __forceinline__ int fragment_at(int row, int k) {
     return (((k >> 5) * 2 + ((k >> 3) & 1)) * 64 + (row ^ piece_of(k)) + 32 * ((k >> 4) & 1)) * 8 + (k & 7);
 }
+// The k at which channel ch of psi and h1 stands, in the order that mg_mlp_chain_bf16 asks W1 and W2 for: a lane half of the matrix core
+// holds channels 8 i + 4 G .. + 3 of a chunk, eight of which in a row are one piece of 16 bytes.
+__device__ __forceinline__ int operand_k(int ch) { return (ch & ~31) + 16 * ((ch >> 2) & 1) + 4 * ((ch >> 3) & 3) + (ch & 3); }
 
-// The two planes of a packed weight (rows of I; PERMUTED: the channels of a chunk in the order that mg_mlp_chain_bf16 asks for) into
-// fragments: [32 rows][16 k][plane][lane][8]
+// The two planes of a packed weight (rows of I) into fragments: [32 rows][16 k][plane][lane][8]
 struct Repack {
     const __bf16* from;
     long plane;
-    int rows, I, permuted;
+    int rows, I;
     __bf16* to;
 };
 struct RepackAll {
@@ -66,14 +67,8 @@ __global__ void __launch_bounds__(256) mlp_chain_repack_kernel(const RepackAll a
     const int lane = (int)(t & 63), plane = (int)(t >> 6) & 1, steps = w.I / 16;
     const long step = t >> 7;
     const int row = 32 * (int)(step / steps) + (lane & 31), s = (int)(step % steps);
-    const __bf16* from = w.from + plane * w.plane + (long)row * w.I + 32 * (s >> 1);
-    bf16x8 v;
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int ch = 16 * (lane >> 5) + 8 * (s & 1) + j;
-        v[j] = from[w.permuted ? 16 * ((ch >> 2) & 1) + 4 * (ch >> 3) + (ch & 3) : ch];
-    }
-    *reinterpret_cast<bf16x8*>(w.to + 8 * t) = v;
+    const __bf16* from = w.from + plane * w.plane + (long)row * w.I + 32 * (s >> 1) + 16 * (lane >> 5) + 8 * (s & 1);
+    *reinterpret_cast<bf16x8*>(w.to + 8 * t) = *reinterpret_cast<const bf16x8*>(from);
 }
 
 // acc[mi] += rows of block mi (from LDS) times 32 weight rows, a step of 16 k at a time; the weights of two steps are in flight.
@@ -226,7 +221,7 @@ mlp_chain_bf16_kernel(const __bf16* __restrict__ X, long R, int I, const __bf16*
         __syncthreads();                                           // (the last stage may lie where psi goes)
         __bf16* psi[4];                                            // of rows q % 4
 #pragma unroll
-        for (int i = 0; i < 4; i++) psi[i] = lds + 2 * half * kStageBlock + fragment_at(4 * G + i, 32 * cb + m);
+        for (int i = 0; i < 4; i++) psi[i] = lds + 2 * half * kStageBlock + fragment_at(4 * G + i, operand_k(32 * cb + m));
         float v[2][16];
 #pragma unroll
         for (int mi = 0; mi < 2; mi++)
@@ -247,17 +242,17 @@ mlp_chain_bf16_kernel(const __bf16* __restrict__ X, long R, int I, const __bf16*
         h.run(lds, kStageBlock, kD / 16);
         __syncthreads();
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int col = 32 * wave + 8 * t + 4 * G;
-            float b[4];
+        for (int t = 0; t < 2; t++) {                              // channels 16 t + 8 (j / 4) + 4 G + j % 4 of the wave's 32
+            const int col = 32 * wave + 16 * t + 4 * G;
+            float b[8];
 #pragma unroll
-            for (int i = 0; i < 4; i++) b[i] = bias_b[col + i];
+            for (int j = 0; j < 8; j++) b[j] = bias_b[col + 8 * (j / 4) + j % 4];
 #pragma unroll
             for (int mi = 0; mi < kBlocks; mi++) {
-                bf16x4 v;
+                bf16x8 v;
 #pragma unroll
-                for (int i = 0; i < 4; i++) v[i] = (__bf16)activate_c<ACT>(h.acc[mi][4 * t + i] + b[i]);
-                *reinterpret_cast<bf16x4*>(lds + mi * 32 * kH + fragment_at(m, col)) = v;
+                for (int j = 0; j < 8; j++) v[j] = (__bf16)activate_c<ACT>(h.acc[mi][8 * t + j] + b[j]);
+                *reinterpret_cast<bf16x8*>(lds + mi * 32 * kH + fragment_at(m, operand_k(col))) = v;
             }
         }
     }
@@ -323,7 +318,7 @@ int mg_mlp_chain_bf16(const void* x, long rows, int dim_in, const void* packed_Y
         const bool planes = dim_in > kPackedDimIn;
         const __bf16 *from_y = static_cast<const __bf16*>(packed_Y), *from_1 = static_cast<const __bf16*>(packed_W1),
                      *from_2 = static_cast<const __bf16*>(packed_W2);
-        const RepackAll all{{{from_1, (long)kH * kD, kH, kD, 1, w1}, {from_2, (long)kH * kH, kH, kH, 1, w2}, {from_y, (long)kD * dim_in, kD, dim_in, 0, y}}};
+        const RepackAll all{{{from_1, (long)kH * kD, kH, kD, w1}, {from_2, (long)kH * kH, kH, kH, w2}, {from_y, (long)kD * dim_in, kD, dim_in, y}}};
         const long most = planes || dim_in < 2 * kH ? (long)kH * kH / 4 : (long)kD * dim_in / 4;
         mlp_chain_repack_kernel<<<dim3((unsigned)ceil_div(most, 256), planes ? 2 : 3), dim3(256), 0, st>>>(all);
         if (int code = check_launch("mlp_chain_repack_kernel")) return code;

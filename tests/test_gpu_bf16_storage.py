@@ -430,3 +430,26 @@ def test_scale_behind_the_summed_scalar_messages(pkg, ops):
         s_psi, _ = ops.mlp_chain_bf16(Y0, P0.reshape(E, 3 * chan), L[0].weight, L[0].bias, L[2].weight, L[2].bias, graph.row_ptr,
                                       graph.src32, N)
     assert torch.equal(got, (s_psi.to(torch.bfloat16).float() * c * 0.1).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("rows,act", [(130, "leaky"), (300, "silu")])
+def test_scalar_message_chain_adds_in_the_order_of_its_operands(ops, rows, act):
+    """The chain against the plain kernels on activations and weights whose channels stand as the entry point asks for W1 and W2: the
+    same products in the same order, so the same bits, row by row (a segment to each)."""
+    g = torch.Generator().manual_seed(rows)
+    act = {"leaky": ops.ACT_LEAKY, "silu": ops.ACT_SILU}[act]
+    x = torch.randn(rows, 96, generator=g).cuda().to(torch.bfloat16)
+    Y = (torch.randn(128, 96, generator=g) / 96 ** 0.5).cuda()
+    W1, W2 = (torch.randn(256, 128, generator=g) / 128 ** 0.5).cuda(), (torch.randn(256, 256, generator=g) / 16).cuda()
+    b1, b2 = torch.randn(256, generator=g).cuda(), torch.randn(256, generator=g).cuda()
+    seg = torch.arange(rows).int().cuda()
+    s_psi, s_h = ops.mlp_chain_bf16(Y, x, W1, b1, W2, b2, ops.segment_row_ptr(seg, rows), seg, rows, act=act)
+    p = torch.arange(16)
+    order = torch.cat([8 * (p // 4) + 4 * half + p % 4 for half in (0, 1)]).cuda()
+
+    def turned(t):
+        return t.view(t.shape[0], -1, 32)[:, :, order].reshape(t.shape).contiguous()
+    psi = ops.tensor_linear_bf16(Y, x)
+    h1 = ops.tensor_linear_bf16(turned(W1), turned(psi), bias=b1, act=act)
+    h2 = ops.tensor_linear_bf16(turned(W2), turned(h1), bias=b2, act=act)
+    assert torch.equal(s_psi, psi.float()) and torch.equal(s_h, h2.float())
