@@ -84,9 +84,6 @@ __global__ void __launch_bounds__(256) bee_geometry_kernel(const float* __restri
     rhat[3 * e + 2] = sz / len;
 }
 
-__device__ __forceinline__ float of_last_lane(float v) {
-    return __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(v), kWave - 1));
-}
 __device__ __forceinline__ long uniform(long v) {
     // the value is the same in every lane: keep it in scalar registers
     const int lo = __builtin_amdgcn_readfirstlane((int)(v & 0xffffffffL));
@@ -349,14 +346,14 @@ bee_message_kernel(const MessageArgs<T> g) {
                 for (int k = 0; k < 45; k++) put_row(o2, lane_bytes, k * row_bytes, (T)s2[k]);
             }
         }
-        if (Y2F || g.node_max) {
+        if (g.node_max) {
             const float mx = wave_max_nonneg_last_lane(active ? largest(s1, s2) : 0.f);
-            if (g.node_max && lane == kWave - 1 && valid) g.node_max[node * chunks + chunk] = mx;
-            if constexpr (Y2F) {
-                __shared__ __attribute__((aligned(16))) float lds[4 * kRank2Share];
-                rank2_linear_of_node_sums<>(s2, of_last_lane(mx), g.split != 0, lds, chunk, chunks, valid, g.y2_packed, g.dim_d,
-                                            g.out_d + node * (long)g.dim_d * 9, g.out_d_accumulate != 0);
-            }
+            if (lane == kWave - 1 && valid) g.node_max[node * chunks + chunk] = mx;
+        }
+        if constexpr (Y2F) {
+            __shared__ __attribute__((aligned(16))) float lds[4 * kRank2Share];
+            rank2_linear_of_node_sums<>(s2, g.split != 0, lds, chunk, chunks, valid, g.y2_packed, g.dim_d,
+                                        g.out_d + node * (long)g.dim_d * 9, g.out_d_accumulate != 0);
         }
     }
 }
@@ -527,13 +524,13 @@ bee_message_ring_kernel(const MessageArgs<T> g) {
                 for (int k = 0; k < 45; k++) put_row(o2, lane_bytes, k * row_bytes, (T)s2[k]);
             }
         }
-        if (Y2F || g.node_max) {
+        if (g.node_max) {
             const float mx = wave_max_nonneg_last_lane(largest(s1, s2));
-            if (g.node_max && lane == kWave - 1 && valid) g.node_max[node * chunks + chunk] = mx;
-            if constexpr (Y2F)
-                rank2_linear_of_node_sums<kShare / 4>(s2, of_last_lane(mx), g.split != 0, reinterpret_cast<float*>(lds), chunk, chunks, valid,
-                                                      g.y2_packed, g.dim_d, g.out_d + node * (long)g.dim_d * 9, g.out_d_accumulate != 0);
+            if (lane == kWave - 1 && valid) g.node_max[node * chunks + chunk] = mx;
         }
+        if constexpr (Y2F)
+            rank2_linear_of_node_sums<kShare / 4>(s2, g.split != 0, reinterpret_cast<float*>(lds), chunk, chunks, valid, g.y2_packed, g.dim_d,
+                                                  g.out_d + node * (long)g.dim_d * 9, g.out_d_accumulate != 0);
     }
 }
 

@@ -203,9 +203,9 @@ __global__ void __launch_bounds__(256) node_products_grad_kernel(long n_nodes, i
 // in one pass: a wave owns (node, 64-channel chunk), a lane one channel; the 45 product values stay in registers
 // and go through rank2_linear_of_node_sums.  Reads the 26 operand rows of a node once (unit stride), writes
 // (node, dim_d, 9); the products themselves are never stored.  For chan = 64, 128 or 256 and dim_d <= 16.
-// 256 channels, 16 outputs, x_d of 16 channels: 780 us at 65 536 nodes, 78 at 8192, 24 at 2048; with the linear on the fp32 matrix
-// cores, x_d through LDS (a broadcast read costs as much as any other) and the scalar and vector products stored before the linear 884, 98
-// and 29.  What bounds it: a wave's chain of loads (of 780 us the linear takes 330, the rank-2 operands 180, the stores 175, and 300 are left
+// 256 channels, 16 outputs, x_d of 16 channels: 775 us at 65 536 nodes, 85 at 8192, 24 at 2048 (870, 114 and 32 where
+// the linear goes the way of fp32); with the linear on the fp32 matrix cores, x_d through LDS (a broadcast read costs as much as any
+// other) and the scalar and vector products stored before the linear 860, 112 and 31.  What bounds it: a wave's chain of loads (of 775 us the linear takes 330, the rank-2 operands 180, the stores 175, and 300 are left
 // without all three), beside 9 GB of weights from the L2.  A chunk's weights in LDS for eight nodes, the chunks of a node in
 // turn: 753 us, but 31 at 2048 nodes, and 1030 with the stores at the end of a chunk, for want of registers; five waves a SIMD 994 us
 // (35 spilled).
@@ -230,7 +230,7 @@ node_rank2_linear_kernel(long n_nodes, int chan, const float* __restrict__ l0,
     const long node = item >> (chunks >> 1);                   // (1, 2 or 4 of them)
     const int chunk = (int)item & (chunks - 1);
     const int c = chunk * kWave + lane;
-    float s2[45], bound = 0.f, lower[18];
+    float s2[45], lower[18];
     if (valid) {
         // x_d is read as scalars below, some lines at a time: all of them are asked for here, beside the other operands
         float touched[9];
@@ -309,18 +309,6 @@ node_rank2_linear_kernel(long n_nodes, int chan, const float* __restrict__ l0,
             lower[6 + 5 * x] = L[3 * x] * v[0] + L[3 * x + 1] * v[1] + L[3 * x + 2] * v[2];
             lower[7 + 5 * x] = cr[x];
         }
-        float ml = fabsf(a), mr = fabsf(b);
-#pragma unroll
-        for (int x = 0; x < 3; x++) {
-            ml = fmaxf(ml, fabsf(u[x]));
-            mr = fmaxf(mr, fabsf(v[x]));
-        }
-#pragma unroll
-        for (int k = 0; k < 9; k++) {
-            ml = fmaxf(ml, fabsf(L[k]));
-            mr = fmaxf(mr, fabsf(R[k]));
-        }
-        bound = 3.0f * ml * mr;                                // (three terms at most)
 #pragma unroll
         for (int x = 0; x < 3; x++) {
             // 212: row x of L crossed with v
@@ -342,8 +330,7 @@ node_rank2_linear_kernel(long n_nodes, int chan, const float* __restrict__ l0,
 #pragma unroll
         for (int k = 0; k < 18; k++) lower[k] = 0.f;
     }
-    bound = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(wave_max_nonneg_last_lane(bound)), kWave - 1));
-    rank2_linear_of_node_sums<>(s2, bound, split != 0, rank2_lds, chunk, chunks, valid, y2_packed, dim_d, out + node * (long)dim_d * 9);
+    rank2_linear_of_node_sums<>(s2, split != 0, rank2_lds, chunk, chunks, valid, y2_packed, dim_d, out + node * (long)dim_d * 9);
     if (P0 && valid) {
         // In the layout of mg_bee_node_products with their maximum per (node, chunk): the operands are in registers once, and the
         // two GEMMs that follow read 18 chan floats per node instead of gathering 26 chan through their operand loads.  Behind everything

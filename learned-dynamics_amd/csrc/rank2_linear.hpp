@@ -8,13 +8,15 @@
 // LDS, from which a lane takes one component at four channels (rows 9 .. 15 of the operand repeat others and are not used).  The
 // waves' partial 9 x 16 results are added through LDS by the first wave of each node.
 //
-// The products are those of f16x2.hpp with the lo lo term (which the matrix cores have time for), scaled per wave by a bound of its
+// The products are those of f16x2.hpp with the lo lo term (which the matrix cores have time for), scaled per wave by the largest of its
 // values and per output by the weight: 40 instructions (16x16x32 in fp16) of 16 cycles.  On the fp32 matrix cores (16x16x4) it is 80 of
 // 32 cycles, and those keep the vector instructions of the other waves waiting (an fp32 matrix instruction and eight multiply-adds
-// beside it take 53 cycles, 34 and 24 by themselves): they remain for values or weights that the pieces cannot carry (infinities,
-// beyond_split) and where fp32 products are asked for.
-// The edge kernel with 256 channels and 16 outputs: 2.07 -> 1.93 ms at 65 536 nodes, 80 -> 74 us at 2048.  Distance from float64 (2-norm,
-// normal values): 1.31e-7 for 1.66e-7 in fp32, and 1.64e-7 without the lo lo term.
+// beside it take 53 cycles, 34 and 24 by themselves): they remain for values or weights that the pieces cannot carry (pieces_fit) and
+// where fp32 products are asked for.
+// The edge kernel with 256 channels, 16 outputs and 20 edges a node: 2.30 -> 2.28 ms at 65 536 nodes, 69.6 -> 65.4 us at 2048.  Distance of
+// a component from float64 (2-norm, normal values): 1.33e-7 for 1.63e-7 in fp32 in the node kernel, 1.38e-7 for 1.74e-7 in the edge
+// kernel, and 1.64e-7 without the lo lo term.  A scale for each component, with no fp32 path for components of unlike size, takes 60
+// instructions and 12 to 18 spilled registers more: 70.5 us for the edge kernel at 2048 nodes, 890 against 775 for the node kernel at 65 536.
 #pragma once
 #include "common.hpp"
 #include "f16x2.hpp"
@@ -54,6 +56,23 @@ __device__ __forceinline__ float wave_max_nonneg_last_lane(float v) {
     x = step(x, std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});   // row_bcast:15
     x = step(x, std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});   // row_bcast:31
     return __uint_as_float(x);
+}
+
+// Whether pieces under one scale can carry the wave's values: none beyond them, and each of the nine components, a sum of its own, no
+// smaller than 2^-12 of the largest value, so that the last bit of a low piece is below 2^-26 of the component's largest.  It is
+// enough that one lane has all nine of that size, which takes one comparison.  bound: the largest |s2| (NaN left out), the same in every lane.
+__device__ __forceinline__ bool pieces_fit(const float (&s2)[45], float& bound) {
+    float most = 0.f, least = __builtin_inff();
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        float v = 0.f;
+#pragma unroll
+        for (int lab = 0; lab < 5; lab++) v = fmaxf(v, fabsf(s2[5 * k + lab]));
+        most = fmaxf(most, v);
+        least = fminf(least, v);
+    }
+    bound = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(wave_max_nonneg_last_lane(most)), kWave - 1));
+    return !beyond_split(bound) && __any(least >= 0x1p-12f * bound);
 }
 
 // a value that is uniform over the wave and never written while the kernel runs, as a scalar load
@@ -167,12 +186,12 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // Called by all four waves of the workgroup (it holds two barriers); valid = false: a wave without an item, whose s2
-// must be zeros.  bound: of |s2| over the wave, the same in every lane.  split: pieces may take the place of fp32 products.
+// must be zeros.  split: pieces may take the place of fp32 products.
 // lds: kRank2Share floats for each wave, SHARE apart, 16-byte aligned.  out: this wave's node, (dim_d, 9);
 // accumulate: the result is added to what out holds.
 template <int SHARE = kRank2Share>
-__device__ __forceinline__ void rank2_linear_of_node_sums(const float (&s2)[45], float bound, bool split, float* lds, int chunk,
-                                                          int chunks, bool valid, const float* __restrict__ y2_packed, int dim_d,
+__device__ __forceinline__ void rank2_linear_of_node_sums(const float (&s2)[45], bool split, float* lds, int chunk, int chunks, bool valid,
+                                                          const float* __restrict__ y2_packed, int dim_d,
                                                           float* __restrict__ out, bool accumulate = false) {
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     float* const tr = lds + wave * SHARE;
@@ -180,7 +199,8 @@ __device__ __forceinline__ void rank2_linear_of_node_sums(const float (&s2)[45],
     const _Float16* const pieces = reinterpret_cast<const _Float16*>(y2_packed + chunks * kRank2Fp32);
     const float iw = reinterpret_cast<const float*>(pieces + chunks * kRank2Pieces)[ci];
     floatx4 d;
-    if (split && !beyond_split(bound) && !__any(iw != iw)) {
+    float bound;
+    if (pieces_fit(s2, bound) && split && !__any(iw != iw)) {
         float inv;
         const float scale = pow2_scale(bound, &inv);
         d = rank2_sums_f16x2<true>(s2, scale, tr, pieces + chunk * kRank2Pieces) * inv * iw;

@@ -176,6 +176,50 @@ def test_rank2_linear_in_pieces_and_in_fp32(ops, chan, dim_d, N, what):
         assert bool(((y.double() - z.double()).abs() <= 2.0 ** -23 * bound)[finite].all())
 
 
+@pytest.mark.parametrize("chan,N", [(64, 9), (256, 6)])
+@pytest.mark.parametrize("what", ["axis 2^-10", "axis 2^-20", "axis 2^-24", "large scalars", "large scalars, no tensors", "one zero"])
+def test_rank2_linear_of_components_of_unlike_size(ops, chan, N, what):
+    """The rank-2 linear inside the edge and the node kernel where the components of a node's products, or ranks of its operands, differ in
+    size: every entry against float64 within 2^-22 of its own sum of |w| |p|: 2^-23 for the linear, as in the test above, and as much for
+    products that another kernel forms (up to three terms, contracted or not).  Of the edge kernel all edges lie along z, so that
+    components without it come from the rank-2 operand alone."""
+    g = torch.Generator().manual_seed(chan + N)
+    dim_d = 16
+    t = [torch.randn(N, *k, chan, generator=g) for k in ((), (3,), (9,), (), (3,), (9,))]
+    W = (torch.randn(dim_d, 5 * chan, generator=g) / (5 * chan) ** 0.5).cuda()
+    edge = [x.clone() for x in t[:3]]
+    if what.startswith("axis"):
+        f = {"10": 2.0 ** -10, "20": 2.0 ** -20, "24": 2.0 ** -24}[what[-2:]]
+        for v in (1, 4):
+            t[v][:, 2] *= f
+            m = torch.ones(3, 3)
+            m[2, :] *= f
+            m[:, 2] *= f
+            t[v + 1] *= m.reshape(1, 9, 1)
+        edge[2] *= f
+    elif what.startswith("large"):
+        t[0] *= 1e6
+        t[3] *= 1e6
+        edge[0] *= 1e6
+        if what.endswith("no tensors"):
+            t[2].zero_()
+            t[5].zero_()
+    else:
+        t[1][:, 2], t[4][:, 2], t[2][:, 6:], t[5][:, 6:] = 0., 0., 0., 0.
+        edge[2].zero_()
+    t, edge = [x.cuda() for x in t], [x.cuda() for x in edge]
+    E = 2 * N
+    row_ptr, dst = (torch.arange(N + 1) * 2).int().cuda(), torch.randint(0, N, (E,), generator=g).int().cuda()
+    enc, rhat = ops.bee_edge_geometry((torch.rand(E, 1, generator=g) * 3 + 1).cuda() * torch.tensor([0., 0., 1.]).cuda(), 6.0)
+    encW, encb = (torch.randn(chan, 8, generator=g) * 0.3).cuda(), torch.randn(chan, generator=g).cuda()
+    for y, p in ((ops.bee_node_products_rank2(*t, W), ops.bee_node_products(*t)[2]),
+                 (ops.bee_message(row_ptr, dst, rhat, enc, *edge, encW, encb, Y2=W)[2],
+                  ops.bee_message(row_ptr, dst, rhat, enc, *edge, encW, encb)[2])):
+        p = p.double().reshape(N, 9, 5 * chan)
+        ref, size = (p @ W.double().t()).transpose(1, 2), (p.abs() @ W.double().abs().t()).transpose(1, 2)
+        assert bool(((y.double() - ref).abs() <= 2.0 ** -22 * size).all())
+
+
 @pytest.mark.parametrize("chan,bf16", [(64, False), (128, False), (256, False), (64, True), (192, True)])
 def test_bee_message_rows_of_every_short_length(ops, chan, bf16):
     """Rows of 0 to 9 and of 33 edges, through LDS (16-byte aligned operands) and through registers (operands 4 bytes off): both do
