@@ -664,12 +664,12 @@ __global__ void __launch_bounds__(256) linear_few_inputs_kernel(const float* __r
 
 // The same for nine components whose outputs lie component by component: a lane owns a channel and forms its nine sums of a row, so
 // that a word of the inputs, read from LDS sixteen bytes at a time, meets nine times fewer instructions.  The sums in the order of
-// the kernel above (the same bits).  vector: a channel's weights are 16-byte pieces.
-// 16 -> 256 channels: 2048 rows 23.0 -> 12.8 us, 1024 rows 16.3 -> 9.8, 3400 rows 28.3 -> 19.1, calls of 8 us at least.  (A wave's inputs
-// as scalar operands instead: 16.8 us, a row waits for four batches of them.)
+// the kernel above (the same bits).  A channel's weights are 16-byte pieces.
+// 16 -> 256 channels: 2048 rows 19.9 -> 10.1 us, 1024 rows 13.6 -> 6.6, 3400 rows 25.0 -> 16.2, one row 3.7 -> 3.2.  (A wave's inputs
+// as scalar operands instead: two thirds more, a row waits for four batches of them.)
 template <int KMAX>
-__global__ void __launch_bounds__(256) linear_few_inputs_by_channel_kernel(const float* __restrict__ W, long so, long si, int vector,
-                                                                           const float* __restrict__ X, long R, int I, int O,
+__global__ void __launch_bounds__(256) linear_few_inputs_by_channel_kernel(const float* __restrict__ W, long so, const float* __restrict__ X,
+                                                                           long R, int I, int O,
                                                                            const float* __restrict__ bias, int act, int accumulate,
                                                                            int tile_rows, float* __restrict__ Y) {
     constexpr int T = 9, kRow = KMAX * T, kMaxRows = 16;
@@ -680,15 +680,10 @@ __global__ void __launch_bounds__(256) linear_few_inputs_by_channel_kernel(const
     const int o = blockIdx.y * 256 + threadIdx.x, o_in = o < O ? o : O - 1;
     float w[KMAX];
     const float* const w_row = W + (long)o_in * so;
-    if (vector) {
 #pragma unroll
-        for (int i = 0; i < KMAX; i += 4) {
-            const float4 v = i < I ? *reinterpret_cast<const float4*>(w_row + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-            w[i] = v.x; w[i + 1] = v.y; w[i + 2] = v.z; w[i + 3] = v.w;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < KMAX; i++) w[i] = i < I ? w_row[(long)i * si] : 0.f;
+    for (int i = 0; i < KMAX; i += 4) {
+        const float4 v = i < I ? *reinterpret_cast<const float4*>(w_row + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+        w[i] = v.x; w[i + 1] = v.y; w[i + 2] = v.z; w[i + 3] = v.w;
     }
     const float b = bias ? bias[o_in] : 0.f;
     for (int k = threadIdx.x; k < rows * kRow; k += 256) {
@@ -725,20 +720,27 @@ constexpr int few_inputs_max(int T) { return T == 1 ? 32 : 16; }
 template <int T>
 int launch_few_inputs(const float* W, long so, long si, const float* X, long R, int I, int O, const float* bias, int act,
                       int accumulate, int y_comp_major, float* Y, hipStream_t st) {
-    if (T == 9 && y_comp_major) {
+    // A lane to a channel where that is faster (us: a thread to each channel and component / a lane to each channel).  16 inputs: from
+    // 128 outputs on, one row 3.7 / 3.0, 2048 rows 12.8 / 8.7, 65 536 179 / 143 (300 outputs 3.7 / 3.2, 20 / 15, 426 / 343), and from 64 on
+    // up to 4096 rows: 2048 9.1 / 7.5, 4096 12.8 / 13.1, but 8192 19.8 / 23.9, where lanes beyond the outputs idle, as they do with 48:
+    // 17.4 / 22.8.  8 and 12 inputs, less to gain: from 128 outputs and 98 304 sums of nine, up to 16 384 rows: 8 -> 128 1024 rows
+    // 6.2 / 4.8, 8 -> 300 8192 rows 28.9 / 24.4, 12 -> 128 1024 rows 6.8 / 5.4, but 12 -> 256 16 rows 3.7 / 4.5, 8 -> 64 8192 rows 12.6 / 18.6,
+    // 8 -> 300 65 536 rows 244 / 264.  Nothing to gain with fewer (4 -> 256 64 rows 2.8 / 3.7, 8192 18.4 / 19.1) nor where a channel's
+    // weights are no 16-byte pieces (9 -> 256 64 rows 3.6 / 4.8).
+    const bool pieces = si == 1 && so % 4 == 0 && I % 4 == 0 && aligned16(W);
+    const bool by_channel = I == 16 ? O >= 128 || (O >= 64 && R <= 4096) : I >= 8 && O >= 128 && R * O >= 98304 && R <= 16384;
+    if (T == 9 && y_comp_major && pieces && by_channel) {
         // tiles of 16 rows, fewer where that would leave CUs without work
         const long blocks = ceil_div(O, 256);
         int rows = 16;
         while (rows > 2 && ceil_div(R, rows) * blocks < 512) rows >>= 1;
         MG_REQUIRE(ceil_div(R, rows) <= 0x7fffffffL && blocks <= 65535, "mg_tensor_linear: grid too large (rows=%ld dim_out=%d)", R, O);
-        const int vector = si == 1 && so % 4 == 0 && I % 4 == 0 && aligned16(W);
         auto launch = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(R, rows), (unsigned)blocks), dim3(256), 0, st, W, so, si, vector, X, R, I, O,
-                               bias, act, accumulate, rows, Y);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(R, rows), (unsigned)blocks), dim3(256), 0, st, W, so, X, R, I, O, bias, act,
+                               accumulate, rows, Y);
             return check_launch("mg_tensor_linear");
         };
-        return I <= 4 ? launch(linear_few_inputs_by_channel_kernel<4>) : I <= 8 ? launch(linear_few_inputs_by_channel_kernel<8>)
-                                                                               : launch(linear_few_inputs_by_channel_kernel<16>);
+        return I == 8 ? launch(linear_few_inputs_by_channel_kernel<8>) : launch(linear_few_inputs_by_channel_kernel<16>);
     }
     // tiles of 64 rows, fewer where that would leave CUs without work
     const long cols = ceil_div((long)O * T, 256);

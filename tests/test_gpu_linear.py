@@ -950,6 +950,13 @@ def test_few_inputs_of_rank_two_by_component_and_by_channel(rows, dim_in, dim_ou
         torch.testing.assert_close(by_channel.cpu().double().reshape(rows, dim_out, 9), ref, rtol=1e-5, atol=1e-6 * dim_in)
 
 
+@pytest.mark.parametrize("rows,dim_in,dim_out", [(1, 16, 63), (1, 16, 64), (767, 8, 128), (768, 8, 128), (900, 12, 127), (769, 12, 128),
+                                                 (5, 16, 513)])
+def test_few_inputs_of_rank_two_beside_the_line_between_their_kernels(rows, dim_in, dim_out):
+    """Channels and sums on either side of where a lane takes a channel of its own: the same bits from both."""
+    test_few_inputs_of_rank_two_by_component_and_by_channel(rows, dim_in, dim_out)
+
+
 @pytest.mark.parametrize("rows, dim_in, dim_out, comps", [
     (1, 288, 64, 1), (33, 256, 256, 1), (95, 544, 40, 1), (31, 1280, 16, 1), (333, 1280, 64, 3), (2050, 160, 70, 1), (1800, 320, 96, 9)])
 def test_reductions_split_over_waves_with_one_chunk_and_several(ops, rows, dim_in, dim_out, comps):
