@@ -199,7 +199,8 @@ class SelfTensProds(nn.Module):
         y_d = y_d.reshape(*rest, dim_d, 3, 3)
         res = (in_a.contiguous(), in_v.contiguous(), in_d.contiguous()) if residual else (None, None, None)
         norms = (self.gn_a, self.gn_v, self.gn_d)
-        if len(rest) == 2 and all(diff.plain_call(gn, TensGroupNorm) for gn in norms):
+        if (len(rest) == 2 and ops.tens_group_norms_supported(*rest, max(dim_a, 3 * dim_v, 9 * dim_d))
+                and all(diff.plain_call(gn, TensGroupNorm) for gn in norms)):
             return tuple(ops.tens_group_norms([(y, gn.groups, gn.gamma.reshape(-1).contiguous(), gn.epsilon, r)
                                                for gn, y, r in zip(norms, (y_a, y_v, y_d), res)]))
         if residual:

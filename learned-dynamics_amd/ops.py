@@ -2397,9 +2397,14 @@ def group_norm(mode, x, groups, gamma, beta=None, eps=1e-5, mul=None, add=None, 
     return out
 
 
+def tens_group_norms_supported(batch, nodes, widest):
+    """tens_group_norms takes rows of `widest` floats (channels x components of the widest tensor)."""
+    return widest <= 65536
+
+
 def tens_group_norms(norms):
     """group_norm(GN_TENSOR, ..) of up to three (x (batch, nodes, chan, (3,)^inds), groups, gamma, eps, res or None) over the same nodes,
-    x and res contiguous, in the two launches of one."""
+    x and res contiguous, in the two launches of one, where tens_group_norms_supported."""
     x, groups, gamma, eps, res = zip(*norms)
     return _ext.tens_norms(x, gamma, res, groups, eps)
 

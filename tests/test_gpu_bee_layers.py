@@ -748,3 +748,18 @@ def test_norms_with_hooks_are_called_one_by_one(pkg):
     assert calls == [1]
     for a, b in zip(together, apart):
         torch.testing.assert_close(a, b, rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("dims", [(65544, 8, 8), (8, 21856, 8), (8, 8, 7288)])
+def test_norms_of_rows_that_one_call_does_not_take(pkg, dims):
+    """SelfTensProds with rows of more than 65 536 floats: its norms are called one by one, as with a hook on one of them."""
+    bl = importlib.import_module("learned-dynamics_amd.bee_layers")
+    torch.manual_seed(6)
+    prods = bl.SelfTensProds(*dims, 16).cuda()
+    x = [torch.randn(1, 3, d, *[3] * k).cuda() for k, d in enumerate(dims)]
+    with torch.no_grad():
+        got = prods(*x, residual=True)
+        hook = prods.gn_v.register_forward_hook(lambda *a: None)
+        want = prods(*x, residual=True)
+        hook.remove()
+    assert all(torch.equal(a, b) and bool(a.isfinite().all()) for a, b in zip(got, want))
