@@ -2398,8 +2398,13 @@ def group_norm(mode, x, groups, gamma, beta=None, eps=1e-5, mul=None, add=None, 
 
 
 def tens_group_norms_supported(batch, nodes, widest):
-    """tens_group_norms takes rows of `widest` floats (channels x components of the widest tensor)."""
-    return widest <= 65536
+    """tens_group_norms takes rows of `widest` floats (channels x components of the widest tensor) and is no slower than the norms one by
+    one.  Its sums have 64 workgroups a box and tensor, which walk over the rows 256 positions at a time, where a norm by itself has 64
+    for each of its groups.  Norms of 128, 64 x 3 and 64 x 9 floats with a residual, us in one call / one by one: one box of 2048 nodes
+    22 / 32, 8192 56 / 55, 65 536 402 / 253; two of 8192 68 / 77, of 16 384 138 / 124; four of 16 384 209 / 216, of 32 768 427 / 406; eight
+    of 16 384 388 / 405.  Of 256 x 9: one box of 1024 nodes 33 / 36, 4096 81 / 68; eight of 8192 646 / 707.  Of 9000 floats a node: one box
+    of 512 nodes 69 / 47, four of 64 60 / 42."""
+    return widest <= 2304 and nodes * widest <= min(batch, 4) << 22
 
 
 def tens_group_norms(norms):

@@ -763,3 +763,20 @@ def test_norms_of_rows_that_one_call_does_not_take(pkg, dims):
         want = prods(*x, residual=True)
         hook.remove()
     assert all(torch.equal(a, b) and bool(a.isfinite().all()) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("batch,nodes,dims", [(1, 7281, (16, 8, 64)), (1, 7282, (16, 8, 64)), (2, 3, (2304, 8, 8)), (2, 3, (2312, 8, 8)), (0, 5, (16, 8, 8))])
+def test_norms_beside_the_line_of_one_call(pkg, batch, nodes, dims):
+    """SelfTensProds on either side of the sizes whose norms are one call: as with the norms called one by one, whose sums of squares
+    are added in another order, in float64."""
+    bl = importlib.import_module("learned-dynamics_amd.bee_layers")
+    torch.manual_seed(nodes)
+    prods = bl.SelfTensProds(*dims, 16).cuda()
+    x = [torch.randn(batch, nodes, d, *[3] * k).cuda() for k, d in enumerate(dims)]
+    with torch.no_grad():
+        got = prods(*x, residual=True)
+        hook = prods.gn_v.register_forward_hook(lambda *a: None)
+        want = prods(*x, residual=True)
+        hook.remove()
+    for a, b in zip(got, want):
+        torch.testing.assert_close(a, b, rtol=1e-6, atol=1e-6)
