@@ -56,6 +56,14 @@ __device__ __forceinline__ void split_pair(float v0, float v1, float s0, float s
     lo = __builtin_convertvector((floatx2{__builtin_fmaf(v0, s0, -(float)hi[0]), __builtin_fmaf(v1, s1, -(float)hi[1])}), halfx2);
 }
 
+// Between a wave's writes to its own LDS and reads of them by other lanes, or those reads and the next writes: LDS keeps the order of
+// one wave, this keeps the compiler to it (the barrier by itself is nothing that memory instructions may not cross)
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 constexpr int kCK = 32;                     // k per chunk (two MFMA steps)
 
 // Packed planes of a weight (O, I): in the order the matrix cores read them.  A block of 32 output rows x one chunk of 32

@@ -81,13 +81,6 @@ __device__ __forceinline__ V scalar_at(const V* p) {
     return *(const __attribute__((address_space(4))) V*)(unsigned long)p;
 }
 
-// between a wave's writes to its own LDS and its reads of them
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // the wave's 9 x 16 sums over its chunk: lane (j = lane % 16, kk = lane / 16), register q: comp 4 kk + q of output j
 __device__ __forceinline__ floatx4 rank2_sums_fp32(const float (&s2)[45], float* tr, int chunk, const float* __restrict__ y2_packed) {
     const int lane = threadIdx.x & (kWave - 1), ci = lane & 15, kk = lane >> 4;

@@ -627,10 +627,10 @@ linear_rows_splitk_f16x2_kernel(const _Float16* __restrict__ Wp, const float* __
             const int r = 8 * j + lane / 8;
             *reinterpret_cast<float4*>(stage + 32 * r + 4 * ((lane & 7) ^ (r / 2 & 7))) = c.a[j];
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
 #pragma unroll
         for (int j = 0; j < 4; j++) c.a[j] = *reinterpret_cast<const float4*>(stage + 32 * m + 4 * ((4 * g + j) ^ (m / 2 & 7)));
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();                                     // (the place is written again)
     };
     auto compute = [&](const Chunk& c) {
 #pragma unroll
