@@ -292,7 +292,7 @@ class MLP(nn.Module):
         """of_linear_summed_over_rows takes x (rows, dim_in of the linear before this MLP) and add_to."""
         L = self.layers
         dim, hidden = L[0].in_features, L[0].out_features
-        return (dim % 256 == 0 and ops.rowsum_into_supported(rows, x.shape[1], dim, x)
+        return (dim % 256 == 0 and hidden % 256 == 0 and ops.rowsum_into_supported(rows, x.shape[1], dim, x)
                 and ops.mlp_rowsum_supported(rows, dim, hidden, x, L[0].bias, L[2].bias, L[4].bias, add_to))
 
     def of_linear_summed_over_rows(self, W, x, bound, row_ptr, n_out, seg, scale=1.0, add_to=None):

@@ -274,6 +274,27 @@ def test_linear_and_mlp_summed_over_segments_as_one_matrix(bee, ops, rows, dim_i
         ops.tensor_linear_f16x2_rowsum(W, x, bound, row_ptr, seg, n_out, into=(S, maxima, 800))
 
 
+def test_messages_whose_hidden_layers_are_no_blocks_of_columns(pkg, bee):
+    """Hidden layers of 320 columns, put in the place of the 512 of an MLP on 256: their sums are no block of a matrix whose maxima are
+    taken over 256 columns, and the messages sum them by themselves.  Against the layers in float64: products of 768 and fewer terms
+    in 22-bit pieces, four layers deep."""
+    gl = importlib.import_module("learned-dynamics_amd.graph_layers")
+    torch.manual_seed(8)
+    N, r0, side = 1024, 5.0, 20.0
+    mod = bee.Messages(r0, 256, 16, 8, 64)
+    for k, (i, o) in {0: (256, 320), 2: (320, 320), 4: (320, 256)}.items():
+        mod.mlp_a.layers[k] = torch.nn.Linear(i, o)
+    mod = mod.cuda()
+    x = torch.randn(1, N, 256).cuda(), torch.randn(1, N, 16, 3).cuda(), torch.randn(1, N, 8, 3, 3).cuda()
+    graph, r_ij = gl.graph_setup(r0, (side,) * 3, (torch.rand(1, N, 3) * side).cuda(), neighbours_max=256, celllist_max=64)
+    assert graph.src.numel() >= 4096
+    with torch.no_grad():
+        got = mod(graph, r_ij, *x)[0]
+    x[0].requires_grad_()                                     # the differentiable path runs every layer on every edge
+    want = mod(graph, r_ij, *x)[0]
+    assert float((got - want.detach()).norm() / want.detach().norm()) <= 2e-6
+
+
 def test_narrow_layers_summed_over_segments_stay_in_fp32(bee, ops, monkeypatch):
     """A linear of 32 columns has fp32 arithmetic: the kernel of 22-bit pieces takes a layer from 64 columns on."""
     x = torch.zeros(5000, 64).cuda()
