@@ -391,7 +391,7 @@ int launch_rows(const float* W, long so, long si, const float* X, long R, int I,
 // the row maxima of |x_p| on the way.  A product's sum is a chain of its own, as of one linear after the other.  Slabs of 32 k in two
 // LDS buffers with the loads of the next two in flight; a wave has MB x NB blocks of B x B, a workgroup 16 to 128 columns of 32 or 64 rows.
 // Bound by the slab in turn (with one slab in flight half as fast) and, unevenly, by the matrix cores: blocks of 16 where there are few
-// columns, which leave none of them empty, and the row count that gives every CU its share.  Five products of 256 channels, us with
+// columns, which leave none of them empty, and the row count that gives every CU its share (of 33 to 64 columns up to 40 960 rows).  Five products of 256 channels, us with
 // blocks of 16 / of 32 in tiles of 128 and 64 rows / in five launches of linear_kernel / bytes at 5 TB/s: 73 728 rows -> 16 85 / 104 /
 // 200 / 76, 18 432 29 / 42, 3000 22 / 40; 24 576 -> 64 55 / 63 / 165 / 26, 900 26 / 37.  Beyond 64 columns the larger blocks read less
 // of LDS for what they multiply: 24 576 x 64 -> 256 20.5 against 23.8.  The error against float64 is the same, 2.9e-7.
@@ -868,7 +868,9 @@ int mg_tensor_linear_products(const float* const* W, long w_stride_o, int produc
     auto run = [&](auto launch) { return launch(weights, w_stride_o, x, rows, dim_in, products, dim_out, y, x_rowmax, st); };
     if (dim_out <= 16) return run(launch_products<16, 4, 1, 1>);
     if (dim_out <= 32) return run(launch_products<16, 4, 1, 2>);
-    if (dim_out <= 64) return run(launch_products<16, 2, 1, 2>);
+    // (both us: five products of 256 -> 40, 12 288 rows 36 / 36, 24 576 50 / 58, 36 864 77 / 80, 49 152 90 / 82, 200 000 367 / 343; three of
+    // 256 -> 64, 36 864 rows 50 / 52, 49 152 59 / 53)
+    if (dim_out <= 64) return rows <= 40960 ? run(launch_products<16, 2, 1, 2>) : run(launch_products<32, 2, 1, 1>);
     return run(launch_products<32, 2, 1, 2>);
 }
 

@@ -1008,3 +1008,9 @@ def test_linears_side_by_side_at_the_edges_of_their_tiles(ops, rows, products, d
     x[0] = float("inf")
     z, _ = ops.row_linears_fwd(x, W, 9, True)
     assert torch.equal(z[1:], y[1:]) and not bool(z[0].isfinite().any())
+
+
+@pytest.mark.parametrize("rows, dim_out", [(40960, 40), (40961, 33), (41001, 64)])
+def test_linears_side_by_side_of_many_rows(ops, rows, dim_out):
+    """Either side of the rows from which 33 to 64 columns go in larger blocks."""
+    test_linears_side_by_side_at_the_edges_of_their_tiles(ops, rows, 2, 32, dim_out)
