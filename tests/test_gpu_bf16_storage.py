@@ -320,10 +320,10 @@ def test_scalar_message_chain_in_one_kernel(ops, kind, dim_in):
     assert not bool(s_psi[empty].any()) and not bool(s_h[empty].any())
 
 
-@pytest.mark.parametrize("rows,dim_in", [(1, 32), (127, 160), (129, 128), (261, 1024), (300, 1056)])
+@pytest.mark.parametrize("rows,dim_in", [(1, 32), (127, 160), (129, 128), (261, 1024), (300, 1056), (133, 8192), (133, 8224)])
 def test_scalar_message_chain_at_the_edges_of_its_tiles(ops, rows, dim_in):
     """Row counts beside the 128 rows of a workgroup, widths beside the 128 k of x that wait in LDS, and a Y on either side of
-    1024, the widest whose fragments the workspace holds (beyond, it is read from its planes).  psi in the order of the plain
+    8192, the widest whose fragments the workspace holds (beyond, it is read from its planes).  psi in the order of the plain
     kernel; bounds of the test above."""
     g = torch.Generator().manual_seed(rows)
     n_seg = 7
