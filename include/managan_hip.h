@@ -290,7 +290,8 @@ int mg_tensor_linear_products(const float* const* W, long w_stride_o, int produc
  *   1  operands split exactly into three bf16 pieces, six bf16 MFMAs per product, fp32
  *      accumulation: same accuracy class as fp32 (dropped terms < 2^-24 |a||b|), ~2.7x the rate;
  *   2  as 1 for callers of mg_tensor_linear*; the host side additionally routes wide plain-row
- *      layers through mg_tensor_linear_f16x2 (below).
+ *      layers through mg_tensor_linear_f16x2 (below), and mg_bee_message_rank2 and
+ *      mg_bee_node_products_rank2 multiply in the same two fp16 pieces where these carry a node's values.
  * Process-wide setting; no counterpart in the reference (its kernel is a plain fp32 dot product,
  * extensions/tensor_ops/tensor_ops_kern.cu:6-42). */
 int mg_set_linear_mode(int mode);
@@ -1032,7 +1033,9 @@ int mg_bee_message(const int* row_ptr, const int* dst, const int* node_order, in
  * which commute with the edge sum of line 252) applied inside the kernel: Y2 (dim_d, 5 chan) = the five Y_lab.W side
  * by side in the label order of S2, packed by mg_bee_pack_rank2_weight into mg_bee_rank2_weight_bytes(chan) bytes;
  * out_d (N, dim_d, 9) = Y2 S2 replaces S2, which is never stored.  For chan = 64, 128 or 256 and dim_d <= 16
- * (mg_bee_message_rank2_supported); the packing has no counterpart in the reference. */
+ * (mg_bee_message_rank2_supported); the packing has no counterpart in the reference.  Products of the linear in mode 2
+ * (mg_set_linear_mode): two fp16 pieces of each operand, scaled per (node, 64 channels) and output, where all nine components
+ * of the sums are of a size (2^-12), and fp32 elsewhere and in the other modes. */
 int mg_bee_message_rank2_supported(int chan, int dim_d);
 int mg_bee_rank2_weight_bytes(int chan, size_t* bytes);
 int mg_bee_pack_rank2_weight(const float* Y2, long row_stride, int chan, int dim_d, float* packed, mg_stream_t stream);
@@ -1043,7 +1046,7 @@ int mg_bee_message_rank2(const int* row_ptr, const int* dst, const int* node_ord
                          float* node_max, float* edge_max, mg_stream_t stream);
 /* The rank-2 part of SelfTensProds.forward (archs/diffuser_atoms15.py:82-94) in one pass over the nodes: the five
  * rank-2 products of l = L_k x_k and r = R_k x_k (component-major operands as for mg_bee_node_products) and their
- * output linears Y_022 .. Y_212, packed as for mg_bee_message_rank2; out_d (N, dim_d, 9).  Same domain.
+ * output linears Y_022 .. Y_212, packed as for mg_bee_message_rank2; out_d (N, dim_d, 9).  Same domain and products.
  * P0 (N,3,chan), P1 (N,3,5,chan) (both or neither; may be NULL): the scalar and vector products as
  * mg_bee_node_products stores them, written in the same pass; node_max (N, chan/64; may be NULL): their partial
  * maxima per node.

@@ -159,7 +159,7 @@ class SelfTensProds(nn.Module):
                                 for k, (lin, x) in enumerate(zip(side, (x_a, x_v, x_d)))], rows)
         ops_in = [p[0] for p in pairs] if not node_pass else list(pairs)
         if node_pass:
-            # one pass over the nodes applies the rank-2 output linear to the products of a node on the fp32 matrix
+            # one pass over the nodes applies the rank-2 output linear to the products of a node on the matrix
             # cores and stores the scalar and vector products (18 chan floats per node) for two plain GEMMs, whose row
             # bounds it emits
             Ys = [_cat_Y(self, labels) for labels in (LABELS_0, LABELS_1, LABELS_2)]

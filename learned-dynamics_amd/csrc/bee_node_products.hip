@@ -203,12 +203,12 @@ __global__ void __launch_bounds__(256) node_products_grad_kernel(long n_nodes, i
 // in one pass: a wave owns (node, 64-channel chunk), a lane one channel; the 45 product values stay in registers
 // and go through rank2_linear_of_node_sums.  Reads the 26 operand rows of a node once (unit stride), writes
 // (node, dim_d, 9); the products themselves are never stored.  For chan = 64, 128 or 256 and dim_d <= 16.
-// 256 channels, 16 outputs, x_d of 16 channels: 775 us at 65 536 nodes, 85 at 8192, 24 at 2048 (870, 114 and 32 where
-// the linear goes the way of fp32); with the linear on the fp32 matrix cores, x_d through LDS (a broadcast read costs as much as any
-// other) and the scalar and vector products stored before the linear 860, 112 and 31.  What bounds it: a wave's chain of loads (of 775 us the linear takes 330, the rank-2 operands 180, the stores 175, and 300 are left
-// without all three), beside 9 GB of weights from the L2.  A chunk's weights in LDS for eight nodes, the chunks of a node in
-// turn: 753 us, but 31 at 2048 nodes, and 1030 with the stores at the end of a chunk, for want of registers; five waves a SIMD 994 us
-// (35 spilled).
+// 256 channels, 16 outputs, x_d of 16 channels: 775 us at 65 536 nodes, 85 at 8192, 24 at 2048 (870, 114 and 32 where the linear goes the
+// way of fp32); with the linear on the fp32 matrix cores, x_d through LDS (a broadcast read costs as much as any other) and the scalar
+// and vector products stored before the linear 860, 112 and 31.  What bounds it: a wave's chain of loads (of 775 us the linear takes
+// 330, the rank-2 operands 180, the stores 175, and 300 are left without all three), beside 9 GB of weights from the L2.  A chunk's
+// weights in LDS for eight nodes, the chunks of a node in turn: 753 us, but 31 at 2048 nodes, and 1030 with the stores at the end of a
+// chunk, for want of registers; five waves a SIMD 994 us (35 spilled).
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
 node_rank2_linear_kernel(long n_nodes, int chan, const float* __restrict__ l0,
                                                                 const float* __restrict__ l1, const float* __restrict__ l2,

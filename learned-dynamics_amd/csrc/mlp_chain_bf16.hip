@@ -316,7 +316,7 @@ int mg_mlp_chain_bf16(const void* x, long rows, int dim_in, const void* packed_Y
         const long tiles = ceil_div(rows, kRows);
         const long grid = ceil_div(tiles, 8) * 8;
         MG_REQUIRE(grid <= 0x7fffffffL, "mg_mlp_chain_bf16: grid too large");
-        // packed weights: planes of ceil(dim_out / 128) * 128 rows.  Their fragments are formed on every call: 4 us
+        // packed weights: planes of ceil(dim_out / 128) * 128 rows.  Their fragments are formed on every call: 5 us
         const bool planes = dim_in > kPackedDimIn;
         const __bf16 *from_y = static_cast<const __bf16*>(packed_Y), *from_1 = static_cast<const __bf16*>(packed_W1),
                      *from_2 = static_cast<const __bf16*>(packed_W2);

@@ -113,8 +113,7 @@ __device__ __forceinline__ floatx4 rank2_sums_fp32(const float (&s2)[45], float*
     }
     return (d0 + d1) + (d2 + d3);
 }
-// pieces: those of the wave's chunk; AHEAD: those of a pair of labels are asked for before its rows are written (from memory, not LDS)
-template <bool AHEAD>
+// pieces: those of the wave's chunk, of a pair of labels asked for before its rows are written (from memory, not LDS)
 __device__ __forceinline__ floatx4 rank2_sums_f16x2(const float (&s2)[45], float scale, float* tr, const _Float16* __restrict__ pieces) {
     const int lane = threadIdx.x & (kWave - 1), ci = lane & 15, kk = lane >> 4;
     float* const hi_rows = tr;
@@ -125,10 +124,8 @@ __device__ __forceinline__ floatx4 rank2_sums_f16x2(const float (&s2)[45], float
 #pragma unroll
     for (int p = 0; p < 2; p++) {
         halfx8 ahead[8];
-        if constexpr (AHEAD) {
 #pragma unroll
-            for (int t = 0; t < 8; t++) ahead[t] = w[(8 * p + t) * 64];
-        }
+        for (int t = 0; t < 8; t++) ahead[t] = w[(8 * p + t) * 64];
 #pragma unroll
         for (int k = 0; k < 9; k++) {
             halfx2 hi, lo;
@@ -140,7 +137,7 @@ __device__ __forceinline__ floatx4 rank2_sums_f16x2(const float (&s2)[45], float
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             const halfx8 xh = *reinterpret_cast<const halfx8*>(hi_rows + from + 4 * t), xl = *reinterpret_cast<const halfx8*>(lo_rows + from + 4 * t);
-            const halfx8 wh = AHEAD ? ahead[2 * t] : w[(8 * p + 2 * t) * 64], wl = AHEAD ? ahead[2 * t + 1] : w[(8 * p + 2 * t + 1) * 64];
+            const halfx8 wh = ahead[2 * t], wl = ahead[2 * t + 1];
             small[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, wh, small[0], 0, 0, 0);
             small[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, wl, small[1], 0, 0, 0);
             large[t & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, wh, large[t & 1], 0, 0, 0);
@@ -149,10 +146,8 @@ __device__ __forceinline__ floatx4 rank2_sums_f16x2(const float (&s2)[45], float
         wave_lds_fence();                                       // the rows are rewritten
     }
     halfx8 ahead[8];
-    if constexpr (AHEAD) {
 #pragma unroll
-        for (int t = 0; t < 8; t++) ahead[t] = w[(16 + t) * 64];
-    }
+    for (int t = 0; t < 8; t++) ahead[t] = w[(16 + t) * 64];
 #pragma unroll
     for (int k = 0; k < 9; k++) {
         const float v = s2[k * 5 + 4];
@@ -163,7 +158,7 @@ __device__ __forceinline__ floatx4 rank2_sums_f16x2(const float (&s2)[45], float
 #pragma unroll
     for (int t = 0; t < 4; t++) {
         const halfx8 x = *reinterpret_cast<const halfx8*>(hi_rows + from + 4 * t);
-        const halfx8 twice = AHEAD ? ahead[2 * t] : w[(16 + 2 * t) * 64], low = AHEAD ? ahead[2 * t + 1] : w[(16 + 2 * t + 1) * 64];
+        const halfx8 twice = ahead[2 * t], low = ahead[2 * t + 1];
         small[t & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, low, small[t & 1], 0, 0, 0);
         large[t & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, twice, large[t & 1], 0, 0, 0);
     }
@@ -196,7 +191,7 @@ __device__ __forceinline__ void rank2_linear_of_node_sums(const float (&s2)[45],
     if (pieces_fit(s2, bound) && split && !__any(iw != iw)) {
         float inv;
         const float scale = pow2_scale(bound, &inv);
-        d = rank2_sums_f16x2<true>(s2, scale, tr, pieces + chunk * kRank2Pieces) * inv * iw;
+        d = rank2_sums_f16x2(s2, scale, tr, pieces + chunk * kRank2Pieces) * inv * iw;
     } else {
         d = rank2_sums_fp32(s2, tr, chunk, y2_packed);
     }
