@@ -32,7 +32,8 @@ constexpr int kStage = 128, kStageBlock = 32 * kStage;            // k of x in L
 constexpr int kStageElems = kRows * kStage;                       // (psi has the place of a stage, h1 that of both)
 constexpr int kStep = 2 * 64 * 8;                                 // elements of a weight's fragments for 16 k: two planes
 // Widest Y that the workspace has room for in fragments, 4 MB of it.  Read from its planes, a line for every row, Y takes 16 384 rows of
-// 1056 54 us and 100 000 175, in fragments 47 and 134; of 2048 92 and 353, 66 and 231.
+// 1056 54 us and 100 000 175, in fragments 47 and 134; of 2048 92 and 353, 66 and 231.  (From 3072 columns on the weights, read for every
+// 128 rows, make some row counts slower than the kernel before, which read them for 256: 40 000 rows of 3072 143 us, there 130.)
 constexpr int kPackedDimIn = 8192;
 
 template <int ACT>
